@@ -27,6 +27,7 @@ from typing import Any, Protocol
 import torch
 
 from . import _lib
+from ._autograd import PositionalFunction
 from .halo import (HaloGeometry, halo_assemble, halo_fold, halo_fold_border_, halo_gather_axis, halo_pack,
                    halo_scatter_add_axis, new_strips, spans_fit_the_strips, strip_table)
 
@@ -1146,7 +1147,7 @@ def _cast_to_autocast_dtype(*tensors):
     return tuple(t if t is None or not t.is_floating_point() else t.to(dt) for t in tensors)
 
 
-class _ConvNd(torch.autograd.Function):
+class _ConvNd(PositionalFunction):
     """Autograd function of the distributed convolution
     (jigsaw/modules/convolution/_conv/functional.py:28-169), HIP kernels inside."""
 
@@ -1163,6 +1164,7 @@ class _ConvNd(torch.autograd.Function):
         x, weight, bias, stride, padding, dilation, spatial_groups, channel_group, config = inputs
         _, x_aug = output
         ctx.mark_non_differentiable(x_aug)
+        ctx.set_materialize_grads(False)  # x_aug has no gradient: no padded tile of zeros for it in the backward
         # the same decision conv_halo_nway took: x_aug is a frame only, so the tile is kept
         ctx.framed = False
         n = config.n_spatial
@@ -1184,6 +1186,8 @@ class _ConvNd(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output, grad_x_aug):  # noqa: D102
+        if grad_output is None:
+            return (None,) * 9
         config = ctx.config
         if ctx.framed:
             x_aug, weight, x_tile = ctx.saved_tensors

@@ -195,6 +195,7 @@ class _ConvTransposeNd(torch.autograd.Function):
             channel_group=channel_group, config=config,
         )
         ctx.mark_non_differentiable(x_aug)
+        ctx.set_materialize_grads(False)  # as in _ConvNd
         ctx.save_for_backward(x_aug, weight)
         ctx.spatial_groups, ctx.channel_group = spatial_groups, channel_group
         ctx.local_in_spatial = tuple(x.shape[-config.n_spatial :])
@@ -204,6 +205,8 @@ class _ConvTransposeNd(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output, grad_x_aug):  # noqa: D102
+        if grad_output is None:
+            return (None,) * 9
         x_aug, weight = ctx.saved_tensors
         config = ctx.config
         need_x, need_w, need_b = ctx.needs_input_grad[:3]

@@ -123,10 +123,13 @@ class _GroupNorm(torch.autograd.Function):
         ctx.save_for_backward(x_norm, rstd, count, w)
         rstd_out, n_out = rstd.unsqueeze(-1).to(cdt), count.unsqueeze(-1).to(cdt)
         ctx.mark_non_differentiable(x_norm, rstd_out, n_out)
+        ctx.set_materialize_grads(False)  # none of the three has a gradient: no tensors of zeros for them
         return y, x_norm, rstd_out, n_out
 
     @staticmethod
     def backward(ctx, grad_output, x_norm_grad, rstd_grad, n_grad):  # noqa: D102
+        if grad_output is None:
+            return (None,) * 6
         x_norm, rstd, count, w = ctx.saved_tensors
         g = grad_output.to(x_norm.dtype).contiguous()
         n, c, s = _dims(x_norm)

@@ -16,6 +16,7 @@ import torch
 import torch.distributed as dist
 
 from . import _lib
+from ._autograd import PositionalFunction
 
 
 def _group_size(group: Any) -> int:
@@ -63,7 +64,7 @@ def _compute_dtype(x: torch.Tensor) -> torch.dtype:
     return x.dtype
 
 
-class _LayerNorm(torch.autograd.Function):
+class _LayerNorm(PositionalFunction):
     """Autograd function of the distributed LayerNorm (HIP kernels inside)."""
 
     @staticmethod
@@ -98,6 +99,7 @@ class _LayerNorm(torch.autograd.Function):
         x, weight, bias, channel_group, eps = inputs
         _, x_norm, w, var = output
         ctx.mark_non_differentiable(x_norm, w, var)
+        ctx.set_materialize_grads(False)  # none of the three has a gradient: no tensors of zeros for them
         ctx.channel_group = channel_group
         ctx.has_bias = bias is not None
         ctx.param_dtypes = (weight.dtype, None if bias is None else bias.dtype)
@@ -107,6 +109,8 @@ class _LayerNorm(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output, x_norm_grad, weight_grad, var_grad):  # noqa: D102
+        if grad_output is None:
+            return (None,) * 5
         x_norm, w, std = ctx.saved_tensors
         g = grad_output.to(x_norm.dtype).contiguous()
         group = ctx.channel_group
