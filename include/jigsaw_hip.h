@@ -531,6 +531,16 @@ int jg_attn_fwd(void* out, float* lse, const void* q, const void* k, const void*
                 const float* bias, int64_t bias_period, float* out_acc,
                 float* lse_acc, int dtype, void* stream);
 
+/* The forward loop of one rank's ring over n_chunks RESIDENT chunks in one call (ring_forward,
+ * _functional/forward.py:160-199, with every chunk here): out (dtype) and lse (fp32) of the queries over all
+ * keys; the running maximum, sum and output stay in registers from the first chunk to the last (the
+ * reference rounds each step's output before it merges it). k, v are HOST arrays of n_chunks device pointers,
+ * read before the call returns. No bias. Covered as jg_attn_bwd_chunks; JG_ERR_UNSUPPORTED otherwise (call
+ * jg_attn_fwd per chunk with the merge). */
+int jg_attn_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v,
+                       int64_t n_chunks, int64_t batch, int64_t sq, int64_t sk, int64_t d, float scale, int dtype,
+                       void* stream);
+
 /* (dq, dk, dv) of one chunk from the GLOBAL out / lse of the ring
  * (cores/math.backward, cores/math.py:81-149): p = exp(scale*q k^T + bias - lse),
  * delta = rowsum(dout*out), ds = p*(dout v^T - delta)*scale, dq = ds k,
@@ -551,8 +561,9 @@ int jg_attn_bwd(void* dq, void* dk, void* dv, const void* dout, const void* q,
  * jg_attn_bwd returns for that chunk), dq the sum of the per-chunk dq, accumulated in fp32 and
  * rounded once (the reference adds the steps in q's dtype, backward.py:184, 269). k, v, dk, dv are
  * HOST arrays of n_chunks device pointers, read before the call returns. No bias.
- * Covered: bf16, d = 64, sq and sk multiples of 128, 1 <= n_chunks <= 16; JG_ERR_UNSUPPORTED
- * otherwise (call jg_attn_bwd per chunk and add the dq). workspace as for jg_attn_bwd. */
+ * Covered: bf16 and fp16, d a multiple of 8 up to 128, any lengths, 1 <= n_chunks <= 16, 16-byte aligned
+ * tensors; JG_ERR_UNSUPPORTED otherwise (call jg_attn_bwd per chunk and add the dq). workspace as for
+ * jg_attn_bwd. */
 int jg_attn_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q,
                        const void* const* k, const void* const* v, int64_t n_chunks, const void* out,
                        const float* lse, int64_t batch, int64_t sq, int64_t sk, int64_t d, float scale,

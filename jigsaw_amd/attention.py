@@ -100,114 +100,44 @@ def _bias_args(bias, batch, sq, sk):
 
 
 # --------------------------------------------------------------------------- #
-# Shapes the MFMA kernels do not take as they are (head sizes other than 64, 96 and 128 -- the
-# "widths" below; fp16 has kernels for 96 and 128 only --, sequence lengths that are not multiples
-# of 128) are brought to them on the host, in bf16 / fp16 and without a bias:
-#   * head size: zero columns are appended to q, k, v (they add nothing to the scores and give
-#     zero output columns);
-#   * queries: zero rows are appended and their results dropped;
-#   * keys, head size below its width: rows are appended whose first spare column holds -c, against
-#     a column of c in q, c = sqrt(30000 / scale) (a value fp16 can hold): their scores are
-#     -30000, their probabilities 0;
-#   * keys, head size equal to its width (no spare column): the multiple of 128 goes through the MFMA kernels, the
-#     remaining keys through the one-thread-per-row kernel, and the two (out, lse) pairs are merged
-#     like two ring steps; the backward treats the two key ranges like two ring chunks, the short
-#     one filled up with zero keys (which the backward's arithmetic ignores by itself).
-# Half of the matrix-core work on zeros is still tens of times faster than the FMA kernel.
+# The 16-bit matrix-core kernels take any lengths and any head size that is a multiple of 8 up to
+# 128, the fp32 ones any lengths at three head sizes, the one-thread-per-row kernels (bias, more
+# batch entries than a grid dimension holds) a few head sizes. Other head sizes get zero columns:
+# they add nothing to the scores and give zero output columns, which are dropped.
 # --------------------------------------------------------------------------- #
-_MASKED_SCORE = -30000.0
-
-
-def _width(d: int, dtype: torch.dtype) -> int:
-    """Head size of the MFMA kernels that take a head of ``d`` columns (fp16: 96 and 128 only)."""
-    return 64 if d <= 64 and dtype == torch.bfloat16 else 96 if d <= 96 else 128
-
-
 _KERNEL_HEAD_SIZES = (8, 16, 32, 64, 96, 128)
-
-
 _F32_MFMA_HEAD_SIZES = (32, 64, 128)
+_MOST_BATCH = 65535
+_MOST_ROWS = 1 << 23  # rows of one head: the kernels address them by 32-bit byte offsets
+
+
+def _mfma16(q, k, bias=None) -> bool:
+    """Whether the 16-bit matrix-core kernels take q against the keys k (their head size padded to a multiple of 8)."""
+    return (bias is None and q.dtype in (torch.bfloat16, torch.float16) and q.shape[-1] <= 128
+            and max(q.shape[-2], k.shape[-2]) <= _MOST_ROWS and math.prod(q.shape[:-2]) <= _MOST_BATCH)
 
 
 def _kernel_head_size(d: int, dtype=None, has_bias: bool = False) -> int:
-    """Smallest head size the kernels are built for that holds ``d`` columns (zero columns change
-    neither scores nor the other outputs); ``d`` itself beyond the largest. fp32 without a bias
-    goes to the sizes of its matrix-core kernels, everything else to those of the
-    one-thread-per-row kernels."""
+    """Smallest head size the kernels beside the 16-bit matrix-core ones are built for that holds ``d`` columns;
+    ``d`` itself beyond the largest. fp32 without a bias goes to the sizes of its matrix-core kernels,
+    everything else to those of the one-thread-per-row kernels."""
     sizes = _F32_MFMA_HEAD_SIZES if dtype == torch.float32 and not has_bias else _KERNEL_HEAD_SIZES
     return next((n for n in sizes if n >= d), d)
 
 
-def _shapeable(q, k, bias) -> bool:
-    d, sq, sk = q.shape[-1], q.shape[-2], k.shape[-2]
-    if bias is not None or q.dtype not in (torch.bfloat16, torch.float16) or d > 128 or sq == 0 or sk < 128:
-        return False
-    return d != _width(d, q.dtype) or sq % 128 != 0 or sk % 128 != 0
+def _padded_head_size(q, k, bias) -> int:
+    d = q.shape[-1]
+    return (d + 7) // 8 * 8 if _mfma16(q, k, bias) else _kernel_head_size(d, q.dtype, bias is not None)
 
 
 def _pad_last(t: torch.Tensor, to: int) -> torch.Tensor:
     return t if t.shape[-1] == to else torch.nn.functional.pad(t, (0, to - t.shape[-1]))
 
 
-def _pad_rows(t: torch.Tensor, to: int) -> torch.Tensor:
-    return t if t.shape[-2] == to else torch.nn.functional.pad(t, (0, 0, 0, to - t.shape[-2]))
-
-
-def _up128(n: int) -> int:
-    return (n + 127) // 128 * 128
-
-
-def _shape_qkv(q, k, v, scale):
-    """q, k, v as the MFMA kernels take them: ``(q, k, v, key ranges)``; a key range is
-    ``(start, stop)`` in the (possibly padded) k / v, the first one a multiple of 128 long."""
-    d, sq, sk = q.shape[-1], q.shape[-2], k.shape[-2]
-    w = _width(d, q.dtype)
-    qp = _pad_rows(_pad_last(q, w), _up128(sq))
-    kp, vp = _pad_last(k, w), _pad_last(v, w)
-    if sk % 128 == 0:
-        return qp, kp, vp, [(0, sk)]
-    if d < w:
-        c = math.sqrt(-_MASKED_SCORE / float(scale))
-        qp[..., d] = c
-        kp, vp = _pad_rows(kp, _up128(sk)), _pad_rows(vp, _up128(sk))
-        kp[..., sk:, d] = -c
-        return qp, kp, vp, [(0, _up128(sk))]
-    main = sk // 128 * 128
-    return qp, kp, vp, [(0, main), (main, sk)]
-
-
-def _shaped_forward(q, k, v, scale):
-    d, sq = q.shape[-1], q.shape[-2]
-    qp, kp, vp, ranges = _shape_qkv(q, k, v, scale)
-    out, lse = _core_forward(qp, kp[..., ranges[0][0]:ranges[0][1], :], vp[..., ranges[0][0]:ranges[0][1], :], scale)
-    if len(ranges) == 2:
-        o2, l2 = _core_forward(qp, kp[..., ranges[1][0]:ranges[1][1], :], vp[..., ranges[1][0]:ranges[1][1], :], scale)
-        rows, w = qp.shape[-2], qp.shape[-1]
-        merged = fused_online_softmax_merge_(out.float().reshape(1, -1, rows, w), lse.reshape(1, -1, rows),
-                                             o2.reshape(1, -1, rows, w), l2.reshape(1, -1, rows), "bhsd")
-        out, lse = merged[0].to(q.dtype).reshape(out.shape), merged[1].reshape(lse.shape)
-    return out[..., :sq, :d].contiguous(), lse[..., :sq].contiguous()
-
-
-def _shaped_backward(grad_out, q, k, v, out, lse, scale):
-    d, sq, sk = q.shape[-1], q.shape[-2], k.shape[-2]
-    qp, kp, vp, ranges = _shape_qkv(q, k, v, scale)
-    rows, w = qp.shape[-2], qp.shape[-1]
-    gp, op = _pad_rows(_pad_last(grad_out, w), rows), _pad_rows(_pad_last(out, w), rows)
-    lp = lse if lse.shape[-1] == rows else torch.nn.functional.pad(lse, (0, rows - lse.shape[-1]))
-    dq, dks, dvs = None, [], []
-    for lo, hi in ranges:
-        # A key range shorter than a tile is filled up with zero keys: with the global out / lse a
-        # zero key adds nothing to dq (its k is zero) and its own dk / dv rows are dropped, so the
-        # backward needs no mask.
-        kj, vj = _pad_rows(kp[..., lo:hi, :], _up128(hi - lo)), _pad_rows(vp[..., lo:hi, :], _up128(hi - lo))
-        dq_j, dk_j, dv_j = _core_backward(gp, qp, kj, vj, op, lp, scale)
-        dq = dq_j.float() if dq is None else dq + dq_j.float()
-        dks.append(dk_j[..., : hi - lo, :])
-        dvs.append(dv_j[..., : hi - lo, :])
-    dk = dks[0] if len(dks) == 1 else torch.cat(dks, dim=-2)
-    dv = dvs[0] if len(dvs) == 1 else torch.cat(dvs, dim=-2)
-    return (dq[..., :sq, :d].to(q.dtype).contiguous(), dk[..., :sk, :d].contiguous(), dv[..., :sk, :d].contiguous())
+def _dense(t: torch.Tensor) -> torch.Tensor:
+    """``t`` contiguous on a 16-byte boundary (a view into a larger tensor may start anywhere)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def core_forward(q, k, v, scale, bias=None, out_acc=None, lse_acc=None, want_out=True):
@@ -216,9 +146,7 @@ def core_forward(q, k, v, scale, bias=None, out_acc=None, lse_acc=None, want_out
     Returns ``(out, lse)`` (``None`` each when ``want_out`` is false).
     """
     _check_qkv(q, k, v)
-    if out_acc is None and lse_acc is None and want_out and _shapeable(q, k, bias):
-        return _shaped_forward(q, k, v, scale)
-    d, dp = q.shape[-1], _kernel_head_size(q.shape[-1], q.dtype, bias is not None)
+    d, dp = q.shape[-1], _padded_head_size(q, k, bias)
     if dp != d and out_acc is None and lse_acc is None:
         out, lse = _core_forward(_pad_last(q, dp), _pad_last(k, dp), _pad_last(v, dp), scale, bias, None, None, want_out)
         return (out[..., :d].contiguous() if want_out else None), lse
@@ -226,7 +154,7 @@ def core_forward(q, k, v, scale, bias=None, out_acc=None, lse_acc=None, want_out
 
 
 def _core_forward(q, k, v, scale, bias=None, out_acc=None, lse_acc=None, want_out=True):
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    q, k, v = _dense(q), _dense(k), _dense(v)
     batch, sq, d = _flat(q)
     sk = int(k.shape[-2])
     bias_t, period = _bias_args(bias, batch, sq, sk)
@@ -257,9 +185,7 @@ def core_backward(grad_out, q, k, v, out, logsumexp, scale, bias=None, want_dbia
     """``(dq, dk, dv[, dbias])`` of one chunk from the global ``out`` / ``logsumexp``."""
     _check_qkv(q, k, v)
     _lib.require_gpu(grad_out, out, logsumexp)
-    if not want_dbias and _shapeable(q, k, bias):
-        return _shaped_backward(grad_out.to(q.dtype), q, k, v, out.to(q.dtype), logsumexp.to(torch.float32), scale)
-    d, dp = q.shape[-1], _kernel_head_size(q.shape[-1], q.dtype, bias is not None)
+    d, dp = q.shape[-1], _padded_head_size(q, k, bias)
     if dp != d:
         res = _core_backward(_pad_last(grad_out, dp), _pad_last(q, dp), _pad_last(k, dp), _pad_last(v, dp),
                              _pad_last(out, dp), logsumexp, scale, bias, want_dbias)
@@ -269,8 +195,8 @@ def core_backward(grad_out, q, k, v, out, logsumexp, scale, bias=None, want_dbia
 
 def _core_backward(grad_out, q, k, v, out, logsumexp, scale, bias=None, want_dbias=False):
     dt = q.dtype
-    grad_out, out = grad_out.to(dt).contiguous(), out.to(dt).contiguous()
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    grad_out, out = _dense(grad_out.to(dt)), _dense(out.to(dt))
+    q, k, v = _dense(q), _dense(k), _dense(v)
     lse = logsumexp.to(torch.float32).contiguous()
     batch, sq, d = _flat(q)
     sk = int(k.shape[-2])
@@ -308,16 +234,13 @@ def backward(grad_out, q, k, v, out, logsumexp, scale, *args, dropout_p=0.0, see
 # per-rank ring loops over local chunks
 # --------------------------------------------------------------------------- #
 def _fused_ok(q, k) -> bool:
-    """Whether one launch attends the chunk AND merges into the running accumulators: the 16-bit MFMA
-    kernels at head sizes 64 / 96 / 128 with lengths in multiples of 128, and the fp32 matrix-core
-    kernel at head sizes 32 / 64 / 128 (any lengths, 16-byte aligned tensors)."""
+    """Whether one launch attends the chunk AND merges into the running accumulators: the 16-bit matrix-core
+    kernels at head sizes that are multiples of 8, the fp32 one at head sizes 32 / 64 / 128 (any lengths,
+    16-byte aligned tensors)."""
     d = q.shape[-1]
-    if q.dtype == torch.float32:
-        return d in (32, 64, 128) and all(t.data_ptr() % 16 == 0 for t in (q, k))
-    return (
-        q.dtype in (torch.bfloat16, torch.float16) and d in (64, 96, 128) and d == _width(d, q.dtype)
-        and q.shape[-2] % 128 == 0 and k.shape[-2] % 128 == 0
-    )
+    if any(t.data_ptr() % 16 for t in (q, k)):
+        return False
+    return d in _F32_MFMA_HEAD_SIZES if q.dtype == torch.float32 else d % 8 == 0 and _mfma16(q, k)
 
 
 def attend_step_(q, kj, vj, scale, out, lse):
@@ -339,13 +262,18 @@ def attend_step_(q, kj, vj, scale, out, lse):
 def ring_forward(q, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.Tensor], scale, rank: int = 0):
     """``(out, lse)`` of one rank's queries over all P chunks, visited in ring order
     ``(rank + step) % P`` (forward_chunk_provider.py:190-192). The accumulator is
-    fp32 and cast to ``q.dtype`` once at the end (forward.py:160-167, 199)."""
+    fp32 and cast to ``q.dtype`` once at the end (forward.py:160-167, 199). 16-bit chunks, all
+    resident here, go through one launch that keeps it in registers (a step's output is then not
+    rounded before it is merged, as it is step by step)."""
     P = len(k_chunks)
+    order = [(rank + step) % P for step in range(P)]
+    one_pass = _resident_forward(q, [k_chunks[j] for j in order], [v_chunks[j] for j in order], scale)
+    if one_pass is not None:
+        return one_pass
     acc = torch.promote_types(q.dtype, torch.float32)
     out = torch.zeros(q.shape, device=q.device, dtype=acc)
     lse = torch.full(q.shape[:-1], float("-inf"), device=q.device, dtype=acc)
-    for step in range(P):
-        j = (rank + step) % P
+    for j in order:
         out, lse = attend_step_(q, k_chunks[j].to(q.dtype), v_chunks[j].to(q.dtype), scale, out, lse)
     return out.to(q.dtype), lse
 
@@ -353,26 +281,46 @@ def ring_forward(q, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.T
 _MAX_CHUNKS_PER_CALL = 16
 
 
-def backward_chunks(dout, q, out, lse, k_chunks, v_chunks, scale):
-    """``(dq, [dk_j], [dv_j])`` over resident chunks in ONE pass (``jg_attn_bwd_chunks``): the dQ
-    kernel walks every chunk with dQ in its registers (one launch, one rounding), the dK/dV kernel
-    takes the chunk as a grid dimension. ``None`` where that entry point does not cover the call
-    (anything but bf16 at head size 64 with lengths that are multiples of 128, up to 16 chunks of
-    one shape)."""
-    P = len(k_chunks)
-    if not 1 <= P <= _MAX_CHUNKS_PER_CALL or len(v_chunks) != P:
+def _resident(q, k_chunks, v_chunks) -> bool:
+    """Whether the one-pass kernels take q against these chunks."""
+    k0 = k_chunks[0]
+    return (len(k_chunks) == len(v_chunks) <= _MAX_CHUNKS_PER_CALL and q.is_cuda and q.shape[-1] % 8 == 0 and _mfma16(q, k0)
+            and k0.shape[:-2] == q.shape[:-2] and k0.shape[-1] == q.shape[-1]
+            and all(t.shape == k0.shape and t.device == q.device for t in (*k_chunks, *v_chunks)))
+
+
+def _pointers(tensors) -> ctypes.Array:
+    return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+
+
+def _resident_forward(q, k_chunks, v_chunks, scale):
+    """``(out, lse)`` over resident chunks in ONE launch (``jg_attn_fwd_chunks``), ``None`` where that does not cover them."""
+    if not k_chunks or not _resident(q, k_chunks, v_chunks):
         return None
-    if q.dtype != torch.bfloat16 or q.shape[-1] != 64 or q.shape[-2] % 128 or k_chunks[0].shape[-2] % 128:
-        return None
-    if any(t.shape != k_chunks[0].shape or t.dtype != q.dtype or t.device != q.device for t in (*k_chunks, *v_chunks)):
-        return None
-    if k_chunks[0].shape[:-2] != q.shape[:-2] or not q.is_cuda:
+    q = _dense(q)
+    ks, vs = [_dense(t.to(q.dtype)) for t in k_chunks], [_dense(t.to(q.dtype)) for t in v_chunks]
+    batch, sq, d = _flat(q)
+    out = torch.empty_like(q)
+    lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)
+    rc = _lib.load().jg_attn_fwd_chunks(
+        _lib.ptr(out), _lib.ptr(lse), _lib.ptr(q), _pointers(ks), _pointers(vs), len(ks), batch, sq, int(ks[0].shape[-2]), d,
+        float(scale), _lib.dtype_code(q.dtype), _lib.stream_ptr(q.device),
+    )
+    _lib.check(rc, "jg_attn_fwd_chunks")
+    return out, lse
+
+
+def _resident_backward(dout, q, out, lse, k_chunks, v_chunks, scale):
+    """``(dq, [dk_j], [dv_j])`` over resident chunks in one pass (``jg_attn_bwd_chunks``), ``None`` where that does not
+    cover them: the dQ kernel walks every chunk with dQ in its registers (one launch, one rounding), the dK/dV
+    kernel takes the chunk as a grid dimension."""
+    if not k_chunks or not _resident(q, k_chunks, v_chunks):
         return None
     _lib.require_gpu(dout, q, out, lse)
-    dout, out, q = dout.to(q.dtype).contiguous(), out.to(q.dtype).contiguous(), q.contiguous()
+    dout, out, q = _dense(dout.to(q.dtype)), _dense(out.to(q.dtype)), _dense(q)
     lse = lse.to(torch.float32).contiguous()
-    ks = [t.contiguous() for t in k_chunks]
-    vs = [t.contiguous() for t in v_chunks]
+    ks, vs = [_dense(t.to(q.dtype)) for t in k_chunks], [_dense(t.to(q.dtype)) for t in v_chunks]
+    P = len(ks)
     batch, sq, d = _flat(q)
     sk = int(ks[0].shape[-2])
     dq = torch.empty_like(q)
@@ -382,15 +330,25 @@ def backward_chunks(dout, q, out, lse, k_chunks, v_chunks, scale):
     lib = _lib.load()
     nbytes = int(lib.jg_attn_bwd_workspace_bytes(batch, sq, sk, d))
     ws = torch.empty(max(nbytes, 4), dtype=torch.uint8, device=q.device)
-    arr = lambda ts: (ctypes.c_void_p * P)(*(t.data_ptr() for t in ts))  # noqa: E731
     rc = lib.jg_attn_bwd_chunks(
-        _lib.ptr(dq), arr(dks), arr(dvs), _lib.ptr(dout), _lib.ptr(q), arr(ks), arr(vs), P, _lib.ptr(out), _lib.ptr(lse),
-        batch, sq, sk, d, float(scale), _lib.dtype_code(q.dtype), _lib.ptr(ws), nbytes, _lib.stream_ptr(q.device),
+        _lib.ptr(dq), _pointers(dks), _pointers(dvs), _lib.ptr(dout), _lib.ptr(q), _pointers(ks), _pointers(vs), P,
+        _lib.ptr(out), _lib.ptr(lse), batch, sq, sk, d, float(scale), _lib.dtype_code(q.dtype), _lib.ptr(ws), nbytes,
+        _lib.stream_ptr(q.device),
     )
-    if rc == -2:
-        return None
     _lib.check(rc, "jg_attn_bwd_chunks")
     return dq, dks, dvs
+
+
+def backward_chunks(dout, q, out, lse, k_chunks, v_chunks, scale):
+    """``(dq, [dk_j], [dv_j])`` over resident chunks in ONE pass (see :func:`ring_backward`). ``None`` for
+    anything but bf16 at head size 64 with lengths that are multiples of 128 and up to 16 chunks of one shape."""
+    if not 1 <= len(k_chunks) <= _MAX_CHUNKS_PER_CALL or len(v_chunks) != len(k_chunks):
+        return None
+    if q.dtype != torch.bfloat16 or q.shape[-1] != 64 or q.shape[-2] % 128 or k_chunks[0].shape[-2] % 128:
+        return None
+    if any(t.dtype != q.dtype for t in (*k_chunks, *v_chunks)):
+        return None
+    return _resident_backward(dout, q, out, lse, k_chunks, v_chunks, scale)
 
 
 def ring_backward(dout, q, out, lse, k_chunks, v_chunks, scale):
@@ -399,9 +357,9 @@ def ring_backward(dout, q, out, lse, k_chunks, v_chunks, scale):
     ``dq`` accumulates over the chunks (backward.py:184, 269; here in fp32, cast to
     ``q.dtype`` at the end — the reference accumulates in ``q.dtype``); the sum of
     dK/dV over the ranks that attended a chunk is the caller's collective. Chunks that are all
-    resident go through one pass (:func:`backward_chunks`) where it covers them."""
+    resident go through one pass (``jg_attn_bwd_chunks``) where it covers them."""
     core = q.dtype
-    one_pass = backward_chunks(dout, q, out, lse, [t.to(core) for t in k_chunks], [t.to(core) for t in v_chunks], scale)
+    one_pass = _resident_backward(dout, q, out, lse, k_chunks, v_chunks, scale)
     if one_pass is not None:
         return one_pass
     dout, out = dout.to(core), out.to(core)

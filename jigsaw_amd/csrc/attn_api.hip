@@ -1,9 +1,9 @@
 // C entry points of the attention core: validate and route to the MFMA flash
-// kernels (bf16 at head size 64; bf16 / fp16 at head sizes 96 and 128) when they cover
-// the problem, to the window or generic kernels otherwise.
+// kernels (bf16 at head size 64; bf16 / fp16 at any head size that is a multiple of 8, up to 128)
+// when they cover the problem, to the window or generic kernels otherwise.
 #include <initializer_list>
 
-#include "jg_common.h"
+#include "attn_chunks.h"
 
 namespace jg {
 bool attn_generic_supported(int d);
@@ -15,24 +15,19 @@ int attn_generic_bwd(void* dq, void* dk, void* dv, float* delta, float* dbias, c
                      const float* lse, long long batch, int sq, int sk, int d, float scale,
                      const float* bias, long long bias_period, int dtype, hipStream_t s);
 bool attn_mfma_fwd_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias);
-int attn_mfma_fwd(void* out, float* lse, const void* q, const void* k, const void* v,
-                  long long batch, int sq, int sk, float scale, float* out_acc, float* lse_acc,
-                  hipStream_t s);
+int attn_mfma_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v, int nchunks,
+                         long long batch, int sq, int sk, float scale, float* out_acc, float* lse_acc, hipStream_t s);
 bool attn_mfma_bwd_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias);
-size_t attn_mfma_bwd_workspace(long long batch, int sq, int sk);
-int attn_mfma_bwd(void* dq, void* dk, void* dv, const void* dout, const void* q, const void* k,
-                  const void* v, const void* out, const float* lse, long long batch, int sq,
-                  int sk, float scale, void* ws, hipStream_t s);
 int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q,
                          const void* const* k, const void* const* v, int nchunks, const void* out, const float* lse,
                          long long batch, int sq, int sk, float scale, void* ws, hipStream_t s);
 bool attn_wide_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias);
-int attn_wide_fwd(void* out, float* lse, const void* q, const void* k, const void* v, long long batch,
-                  int sq, int sk, int d, int dtype, float scale, float* out_acc, float* lse_acc,
-                  hipStream_t s);
-int attn_wide_bwd(void* dq, void* dk, void* dv, const void* dout, const void* q, const void* k,
-                  const void* v, const void* out, const float* lse, long long batch, int sq, int sk,
-                  int d, int dtype, float scale, void* ws, hipStream_t s);
+int attn_wide_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v, int nchunks,
+                         long long batch, int sq, int sk, int d, int dtype, float scale, float* out_acc, float* lse_acc,
+                         hipStream_t s);
+int attn_wide_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q,
+                         const void* const* k, const void* const* v, int nchunks, const void* out, const float* lse,
+                         long long batch, int sq, int sk, int d, int dtype, float scale, void* ws, hipStream_t s);
 bool attn_f32_mfma_fwd_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias);
 int attn_f32_mfma_fwd(void* out, float* lse, const void* q, const void* k, const void* v, long long batch, int sq,
                       int sk, int d, float scale, float* out_acc, float* lse_acc, hipStream_t s);
@@ -68,6 +63,23 @@ bool aligned16(std::initializer_list<const void*> ptrs) {
     if ((reinterpret_cast<uintptr_t>(q) & 15) != 0) return false;
   return true;
 }
+
+// Host arrays of n device pointers, one per chunk.
+typedef std::initializer_list<const void* const*> ChunkArrays;
+int check_chunks(const char* who, int64_t n, ChunkArrays arrays) {
+  if (n > jg::ATTN_MAX_CHUNKS) JG_FAIL(JG_ERR_UNSUPPORTED, "%s: at most %d chunks a call, got %lld", who, jg::ATTN_MAX_CHUNKS, (long long)n);
+  for (const void* const* a : arrays) {
+    JG_REQUIRE(a, "%s: NULL pointer", who);
+    for (int64_t c = 0; c < n; ++c) JG_REQUIRE(a[c], "%s: NULL pointer for chunk %lld", who, (long long)c);
+  }
+  return JG_OK;
+}
+bool chunks_aligned16(int64_t n, ChunkArrays arrays) {
+  for (const void* const* a : arrays)
+    for (int64_t c = 0; c < n; ++c)
+      if (!aligned16({a[c]})) return false;
+  return true;
+}
 }  // namespace
 
 extern "C" int jg_attn_fwd(void* out, float* lse, const void* q, const void* k, const void* v,
@@ -86,14 +98,14 @@ extern "C" int jg_attn_fwd(void* out, float* lse, const void* q, const void* k, 
   if (batch == 0 || sq == 0) return JG_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (jg::attn_mfma_fwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr))
-    return jg::attn_mfma_fwd(out, lse, q, k, v, batch, (int)sq, (int)sk, scale, out_acc, lse_acc, s);
-  if (jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr) &&
-      aligned16({out, q, k, v, out_acc}))
-    return jg::attn_wide_fwd(out, lse, q, k, v, batch, (int)sq, (int)sk, (int)d, dtype, scale, out_acc,
-                             lse_acc, s);
+    return jg::attn_mfma_fwd_chunks(out, lse, q, &k, &v, 1, batch, (int)sq, (int)sk, scale, out_acc, lse_acc, s);
   if (out_acc == nullptr && jg::attn_window_supported(batch, (int)sq, (int)sk, (int)d, dtype) &&
       aligned16({out, q, k, v, bias}))
     return jg::attn_window_fwd(out, lse, q, k, v, batch, scale, bias, bias_period, s);
+  if (jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr) &&
+      aligned16({out, q, k, v, out_acc}))
+    return jg::attn_wide_fwd_chunks(out, lse, q, &k, &v, 1, batch, (int)sq, (int)sk, (int)d, dtype, scale, out_acc,
+                                    lse_acc, s);
   if (jg::attn_f32_mfma_fwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr) &&
       aligned16({out, q, k, v, out_acc}))
     return jg::attn_f32_mfma_fwd(out, lse, q, k, v, batch, (int)sq, (int)sk, (int)d, scale, out_acc, lse_acc, s);
@@ -101,8 +113,8 @@ extern "C" int jg_attn_fwd(void* out, float* lse, const void* q, const void* k, 
     JG_FAIL(JG_ERR_UNSUPPORTED, "%s: head size %lld not in {8, 16, 32, 64, 96, 128}", who, (long long)d);
   if (out_acc != nullptr)
     JG_FAIL(JG_ERR_UNSUPPORTED,
-            "%s: the fused merge needs an MFMA path (bf16 with d in {64, 96, 128} or fp16 with d in {96, 128},"
-            " sq %% 128 == 0, sk %% 128 == 0; fp32 with d in {32, 64, 128}, no bias);"
+            "%s: the fused merge needs an MFMA path (bf16 or fp16 with d a multiple of 8 up to 128,"
+            " fp32 with d in {32, 64, 128}, no bias, 16-byte aligned tensors);"
             " call jg_lse_merge after the core instead", who);
   rc = jg::attn_generic_fwd(out, lse, q, k, v, batch, (int)sq, (int)sk, (int)d, scale, bias,
                             bias_period, dtype, s);
@@ -133,19 +145,18 @@ extern "C" int jg_attn_bwd(void* dq, void* dk, void* dv, const void* dout, const
     JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, workspace_bytes,
             jg_attn_bwd_workspace_bytes(batch, sq, sk, d));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dbias == nullptr &&
-      jg::attn_mfma_bwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr))
-    return jg::attn_mfma_bwd(dq, dk, dv, dout, q, k, v, out, lse, batch, (int)sq, (int)sk, scale,
-                             workspace, s);
-  if (dbias == nullptr &&
-      jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr) &&
-      aligned16({dq, dk, dv, dout, q, k, v, out}))
-    return jg::attn_wide_bwd(dq, dk, dv, dout, q, k, v, out, lse, batch, (int)sq, (int)sk, (int)d,
-                             dtype, scale, workspace, s);
+  if (dbias == nullptr && jg::attn_mfma_bwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr))
+    return jg::attn_mfma_bwd_chunks(dq, &dk, &dv, dout, q, &k, &v, 1, out, lse, batch, (int)sq, (int)sk, scale,
+                                    workspace, s);
   if (jg::attn_window_supported(batch, (int)sq, (int)sk, (int)d, dtype) &&
       aligned16({dq, dk, dv, dout, q, k, v, out, bias, dbias}))
     return jg::attn_window_bwd(dq, dk, dv, dbias, dout, q, k, v, out, lse, batch, scale, bias,
                                bias_period, s);
+  if (dbias == nullptr &&
+      jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr) &&
+      aligned16({dq, dk, dv, dout, q, k, v, out}))
+    return jg::attn_wide_bwd_chunks(dq, &dk, &dv, dout, q, &k, &v, 1, out, lse, batch, (int)sq, (int)sk, (int)d,
+                                    dtype, scale, workspace, s);
   if (dbias == nullptr && jg::attn_f32_mfma_bwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr) &&
       aligned16({dq, dk, dv, dout, q, k, v, out}))
     return jg::attn_f32_mfma_bwd(dq, dk, dv, dout, q, k, v, out, lse, batch, (int)sq, (int)sk, (int)d, scale,
@@ -157,6 +168,27 @@ extern "C" int jg_attn_bwd(void* dq, void* dk, void* dv, const void* dout, const
                               s);
 }
 
+extern "C" int jg_attn_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v,
+                                  int64_t n_chunks, int64_t batch, int64_t sq, int64_t sk, int64_t d, float scale,
+                                  int dtype, void* stream) {
+  const char* who = "jg_attn_fwd_chunks";
+  int rc = check_shape(who, batch, sq, sk, d, scale, dtype);
+  if (rc) return rc;
+  JG_REQUIRE(n_chunks >= 1, "%s: n_chunks must be at least 1", who);
+  JG_REQUIRE(out && lse && q, "%s: NULL pointer", who);
+  rc = check_chunks(who, n_chunks, {k, v});
+  if (rc) return rc;
+  if (batch == 0 || sq == 0) return JG_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (jg::attn_mfma_fwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, false))
+    return jg::attn_mfma_fwd_chunks(out, lse, q, k, v, (int)n_chunks, batch, (int)sq, (int)sk, scale, nullptr, nullptr, s);
+  if (jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, false) && aligned16({out, q}) &&
+      chunks_aligned16(n_chunks, {k, v}))
+    return jg::attn_wide_fwd_chunks(out, lse, q, k, v, (int)n_chunks, batch, (int)sq, (int)sk, (int)d, dtype, scale,
+                                    nullptr, nullptr, s);
+  JG_FAIL(JG_ERR_UNSUPPORTED, "%s: bf16 or fp16, d a multiple of 8 up to 128, 16-byte aligned tensors", who);
+}
+
 extern "C" int jg_attn_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q,
                                   const void* const* k, const void* const* v, int64_t n_chunks, const void* out,
                                   const float* lse, int64_t batch, int64_t sq, int64_t sk, int64_t d, float scale,
@@ -165,15 +197,20 @@ extern "C" int jg_attn_bwd_chunks(void* dq, void* const* dk, void* const* dv, co
   int rc = check_shape(who, batch, sq, sk, d, scale, dtype);
   if (rc) return rc;
   JG_REQUIRE(n_chunks >= 1, "%s: n_chunks must be at least 1", who);
-  JG_REQUIRE(dq && dk && dv && dout && q && k && v && out && lse, "%s: NULL pointer", who);
-  if (n_chunks > 16 || !jg::attn_mfma_bwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, false))
-    JG_FAIL(JG_ERR_UNSUPPORTED, "%s: bf16, d = 64, sq and sk multiples of 128 and at most 16 chunks", who);
-  for (int64_t c = 0; c < n_chunks; ++c)
-    JG_REQUIRE(k[c] && v[c] && dk[c] && dv[c], "%s: NULL pointer for chunk %lld", who, (long long)c);
+  JG_REQUIRE(dq && dout && q && out && lse, "%s: NULL pointer", who);
+  rc = check_chunks(who, n_chunks, {k, v, dk, dv});
+  if (rc) return rc;
   if (batch == 0 || sq == 0) return JG_OK;
   if (workspace == nullptr || workspace_bytes < jg_attn_bwd_workspace_bytes(batch, sq, sk, d))
     JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, workspace_bytes,
             jg_attn_bwd_workspace_bytes(batch, sq, sk, d));
-  return jg::attn_mfma_bwd_chunks(dq, dk, dv, dout, q, k, v, (int)n_chunks, out, lse, batch, (int)sq, (int)sk, scale,
-                                  workspace, static_cast<hipStream_t>(stream));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (jg::attn_mfma_bwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, false))
+    return jg::attn_mfma_bwd_chunks(dq, dk, dv, dout, q, k, v, (int)n_chunks, out, lse, batch, (int)sq, (int)sk, scale,
+                                    workspace, s);
+  if (jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, false) && aligned16({dq, dout, q, out}) &&
+      chunks_aligned16(n_chunks, {k, v, dk, dv}))
+    return jg::attn_wide_bwd_chunks(dq, dk, dv, dout, q, k, v, (int)n_chunks, out, lse, batch, (int)sq, (int)sk, (int)d,
+                                    dtype, scale, workspace, s);
+  JG_FAIL(JG_ERR_UNSUPPORTED, "%s: bf16 or fp16, d a multiple of 8 up to 128, 16-byte aligned tensors", who);
 }

@@ -34,11 +34,20 @@
 //   third grid dimension of the dK/dV kernel. The chunk pointers travel in the kernel-argument
 //   segment (first parameter), where a wavefront reads entry c with scalar loads.
 //
+//   RAGGED (sq or sk no multiple of 128): rows of a transfer clamped to the tensor's last one, resident rows
+//   clamped when read and dropped when written; keys past the end get the score -inf (dQ kernel), queries past
+//   the end the lse +inf (dK/dV kernel), so that their probabilities are 0.
+//
 // Reference behaviour restated here:
 //   jigsaw/modules/attention/_functional/cores/math.py:125-149
-#include "jg_common.h"
+#include "attn_chunks.h"
 
 namespace {
+
+using jg::BlockOf;
+using jg::ChunkTable;
+using jg::block_of;
+using jg::chunk_entry;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -68,6 +77,10 @@ __device__ __forceinline__ bf16x8 lds_frag(const unsigned char* p) {
 // offset, the LDS address of the 1 KB block in M0. (With the compiler's own form of this load
 // it orders every later LDS read behind ALL outstanding transfers, also those of the tile
 // after next; the kernels order reads and transfers themselves, by their waits and barriers.)
+// the same for rows first_row + 0..7 of a tensor of `rows` rows, clamped to its last one
+__device__ __forceinline__ uint32_t dma_clamped_offset(int lane, int first_row, int rows) {
+  return (uint32_t)min(first_row + (lane >> 3), rows - 1) * ROWB + (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4);
+}
 __device__ __forceinline__ uint32_t dma_lane_offset(int lane) {
   return (uint32_t)((lane >> 3) * ROWB + (((lane & 7) ^ (lane >> 3)) << 4));
 }
@@ -120,49 +133,6 @@ __device__ __forceinline__ bf16x8 pack8(const float* e) {
   return pk;
 }
 
-// Workgroup -> (batch entry, row block). Consecutive workgroup ids go to the 8 XCDs in turn; each
-// XCD is given a contiguous range of (batch entry, block) pairs, so the workgroups that stream the
-// same K / V (or Q / dO) share one L2 instead of every L2 holding every head. Falls back to the
-// plain order when the count does not divide.
-struct BlockOf {
-  long long bh;
-  int blk;
-  int chunk;
-};
-// gridDim = (row blocks, batch entries, chunks). The flat order is (batch entry, chunk, block), so the
-// workgroups of one XCD's range stream the Q / dO (or K / V) of the same few batch entries.
-__device__ __forceinline__ BlockOf block_of() {
-  const unsigned nblk = gridDim.x, nch = gridDim.z, total = gridDim.x * gridDim.y * gridDim.z;
-  unsigned id = (blockIdx.y * nch + blockIdx.z) * nblk + blockIdx.x;
-  if ((total & 7u) == 0) id = (id & 7u) * (total >> 3) + (id >> 3);
-  BlockOf b;
-  b.blk = (int)(id % nblk);
-  id /= nblk;
-  b.chunk = (int)(id % nch);
-  b.bh = id / nch;
-  return b;
-}
-
-constexpr int MAX_CHUNKS = 16;
-// Chunk c: k[c], v[c] (batch, sk, 64) and where its gradients go. FIRST kernel parameter: entry c is
-// read from the kernel-argument segment by its offset (a by-value struct indexed with a run-time
-// value would otherwise be copied to private memory lane by lane).
-struct ChunkTable {
-  const uint16_t* k[MAX_CHUNKS];
-  const uint16_t* v[MAX_CHUNKS];
-  uint16_t* dk[MAX_CHUNKS];
-  uint16_t* dv[MAX_CHUNKS];
-};
-__device__ __forceinline__ const char* chunk_entry(int which, int c) {  // which: 0 k, 1 v, 2 dk, 3 dv; c wave-uniform
-#if defined(__HIP_DEVICE_COMPILE__)
-  const char* const* kt = (const char* const*)__builtin_amdgcn_kernarg_segment_ptr();
-  return kt[which * MAX_CHUNKS + c];
-#else
-  (void)which; (void)c;
-  return nullptr;
-#endif
-}
-
 struct BwdArgs {
   const uint16_t* dout;
   const uint16_t* q;
@@ -187,6 +157,7 @@ constexpr int DQ_LDS = 2 * DQ_HALF;         // 131072 (and at least 4 x 32 x 64 
 #define JG_GROUP_MFMA 0x008
 #define JG_GROUP_DS_READ 0x100
 
+template <bool RAGGED>
 __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks, BwdArgs p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x;
@@ -198,19 +169,20 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
   const int q0 = where.blk * BR + qb * 32;
   // every chunk is cut in two key halves (one per wavefront group); a half's tiles of all chunks
   // form one stream of ntiles tiles
-  const int khalf = p.sk >> 1;
-  const int tiles_per_chunk = khalf / BT;
+  const int tiles_per_chunk = (p.sk + 2 * BT - 1) / (2 * BT);
   const int ntiles = tiles_per_chunk * p.nchunks;
   const float c2 = p.scale * LOG2E;
-  const long long qi = b * p.sq + q0 + ln;
+  const bool q_live = !RAGGED || q0 + ln < p.sq;
+  const long long qi = b * p.sq + (q_live ? q0 + ln : p.sq - 1);
 
   unsigned char* lds = smem + ks * DQ_HALF;
   // this wavefront moves rows 16 qb .. 16 qb + 15 of the K tile and of the V tile of its half
   const int ks_u = __builtin_amdgcn_readfirstlane(ks), qb_u = __builtin_amdgcn_readfirstlane(qb);
-  const long long half_off = 2 * ((b * p.sk + (long long)ks_u * khalf) * D) + 16 * qb_u * ROWB;  // bytes into a chunk
+  const long long chunk_off = 2 * (b * p.sk * (long long)D);  // bytes into a chunk
+  const int row_first = ks_u * tiles_per_chunk * BT + 16 * qb_u;
   int ld_chunk = 0, ld_tile = 0;  // the load cursor: tiles are requested in stream order
-  const char* kdma = chunk_entry(0, 0) + half_off;
-  const char* vdma = chunk_entry(1, 0) + half_off;
+  const char* kdma = chunk_entry(0, 0) + chunk_off;
+  const char* vdma = chunk_entry(1, 0) + chunk_off;
   const uint32_t dma_off = dma_lane_offset(lane);
   const uint32_t lds_dma = lds_address(smem) + (uint32_t)(ks_u * DQ_HALF + 16 * qb_u * ROWB);
   const int tr_off[2] = {tr_lane_offset(lane, 0), tr_lane_offset(lane, 1)};
@@ -221,17 +193,26 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
 
   // K and V of tile t straight into its buffer (free since the barrier that ended the tile before)
   auto issue_loads = [&](int t) {  // called with t = 0, 1, 2, ... in turn
-    const long long off = (long long)ld_tile * NAT;
     const uint32_t dst = lds_dma + (uint32_t)((t & (NBUF - 1)) * DQ_BUF);
-    dma_1k(kdma + off, dma_off, dst);
-    dma_1k(kdma + off + 8 * ROWB, dma_off, dst + 8 * ROWB);
-    dma_1k(vdma + off, dma_off, dst + NAT);
-    dma_1k(vdma + off + 8 * ROWB, dma_off, dst + NAT + 8 * ROWB);
+    const int row = row_first + ld_tile * BT;
+    if (RAGGED) {
+      const uint32_t o0 = dma_clamped_offset(lane, row, p.sk), o1 = dma_clamped_offset(lane, row + 8, p.sk);
+      dma_1k(kdma, o0, dst);
+      dma_1k(kdma, o1, dst + 8 * ROWB);
+      dma_1k(vdma, o0, dst + NAT);
+      dma_1k(vdma, o1, dst + NAT + 8 * ROWB);
+    } else {
+      const long long off = (long long)row * ROWB;
+      dma_1k(kdma + off, dma_off, dst);
+      dma_1k(kdma + off + 8 * ROWB, dma_off, dst + 8 * ROWB);
+      dma_1k(vdma + off, dma_off, dst + NAT);
+      dma_1k(vdma + off + 8 * ROWB, dma_off, dst + NAT + 8 * ROWB);
+    }
     if (++ld_tile == tiles_per_chunk && ld_chunk + 1 < p.nchunks) {
       ld_tile = 0;
       ++ld_chunk;
-      kdma = chunk_entry(0, ld_chunk) + half_off;
-      vdma = chunk_entry(1, ld_chunk) + half_off;
+      kdma = chunk_entry(0, ld_chunk) + chunk_off;
+      vdma = chunk_entry(1, ld_chunk) + chunk_off;
     }
   };
   auto tiles_landed = [&]() {
@@ -258,7 +239,7 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
       for (int i = 0; i < 8; ++i) dl += (float)dof[c][i] * (float)of[i];
     }
     delta = dl + __shfl_xor(dl, 32, 64);
-    if (ks == 0 && kg == 0) p.delta[qi] = delta;
+    if (ks == 0 && kg == 0 && q_live) p.delta[qi] = delta;
   }
   const float lse2 = p.lse[qi] * LOG2E;
   f32x16 minus_delta;
@@ -306,7 +287,20 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
         dq[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(kn, tr_off[nb], sb * 32 + 16 * t), ds_prev[t], dq[nb], 0, 0, 0);
   };
   // one step of the pipeline: A of (k_next, sb_next), B of the current block, C of (k_prev, sb_prev)
+  int keys_left = p.sk - ks_u * tiles_per_chunk * BT, tile_at = 0;  // RAGGED: keys from the current block's first one on
   auto step = [&](const unsigned char* k_next, int sb_next, const unsigned char* k_prev, int sb_prev, bool ahead) {
+    if (RAGGED) {
+      if (keys_left < 32) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (8 * (i >> 2) + 4 * kg + (i & 3) >= keys_left) s_cur[i] = -INFINITY;
+      }
+      keys_left -= 32;
+      if (++tile_at == 2 * tiles_per_chunk) {  // the next block opens the next chunk
+        tile_at = 0;
+        keys_left += tiles_per_chunk * BT;
+      }
+    }
     f32x16 s_n, dp_n;
     if (ahead) scores(k_next, sb_next, s_n, dp_n);
     bf16x8 ds_now[2];
@@ -366,7 +360,7 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
       for (int i = 0; i < 16; ++i) xo[(nb * 16 + i) * 64 + lane] = dq[nb][i];
   }
   __syncthreads();
-  if (ks == 1) return;
+  if (ks == 1 || !q_live) return;
 #pragma unroll
   for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
@@ -399,6 +393,7 @@ constexpr int DKV_SHARE = BT / DKV_KB;                // rows of a streamed tile
 static_assert(DKV_LDS >= DKV_KB * 64 * 64 * 4, "the hand-over of the partial dK / dV reuses the tile buffers");
 static_assert(64 * DKV_KB >= 2 * BT, "one thread of a half per statistic");
 
+template <bool RAGGED>
 __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void attn_bwd_dkv_kernel(ChunkTable chunks, BwdArgs p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x;
@@ -409,40 +404,47 @@ __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void at
   const BlockOf where = block_of();
   const long long b = where.bh;
   const int k0 = where.blk * DKV_ROWS + kb * 32;
-  const int qhalf = p.sq >> 1;
-  const int ntiles = qhalf / BT;
+  const int ntiles = (p.sq + 2 * BT - 1) / (2 * BT);
   const float c2 = p.scale * LOG2E;
-  const long long ki = b * p.sk + k0 + ln;
+  const bool k_live = !RAGGED || k0 + ln < p.sk;
+  const long long ki = b * p.sk + (k_live ? k0 + ln : p.sk - 1);
 
   unsigned char* lds = smem + qs * (2 * DKV_HALF);  // two buffers: Q tile, dO tile, stats
-  const long long qrow0 = b * p.sq + (long long)qs * qhalf;
+  const int half_row = qs * ntiles * BT;  // first query of this half
   // this wavefront moves its share of the rows of the Q tile and of the dO tile of its half
   const int qs_u = __builtin_amdgcn_readfirstlane(qs), kb_u = __builtin_amdgcn_readfirstlane(kb);
-  const long long qrow0_u = b * p.sq + (long long)qs_u * qhalf;
-  const char* qdma = reinterpret_cast<const char*>(p.q + qrow0_u * D) + DKV_SHARE * kb_u * ROWB;
-  const char* ddma = reinterpret_cast<const char*>(p.dout + qrow0_u * D) + DKV_SHARE * kb_u * ROWB;
+  const int row_first = qs_u * ntiles * BT + DKV_SHARE * kb_u;
+  const char* qdma = reinterpret_cast<const char*>(p.q + b * p.sq * D);
+  const char* ddma = reinterpret_cast<const char*>(p.dout + b * p.sq * D);
   const uint32_t dma_off = dma_lane_offset(lane);
   const uint32_t lds_dma = lds_address(smem) + (uint32_t)(qs_u * (2 * DKV_HALF) + DKV_SHARE * kb_u * ROWB);
   const int tr_off[2] = {tr_lane_offset(lane, 0), tr_lane_offset(lane, 1)};
 
   float st_reg = 0.0f;
   auto issue_loads = [&](int t, int buf) {
-    const long long off = (long long)t * NAT;
     const uint32_t dst = lds_dma + (uint32_t)(buf * DKV_HALF);
 #pragma unroll
     for (int r = 0; r < DKV_SHARE; r += 8) {
-      dma_1k(qdma + off + r * ROWB, dma_off, dst + r * ROWB);
-      dma_1k(ddma + off + r * ROWB, dma_off, dst + NAT + r * ROWB);
+      const int row = row_first + t * BT + r;
+      const long long off = RAGGED ? 0 : (long long)row * ROWB;
+      const uint32_t lane_off = RAGGED ? dma_clamped_offset(lane, row, p.sq) : dma_off;
+      dma_1k(qdma + off, lane_off, dst + r * ROWB);
+      dma_1k(ddma + off, lane_off, dst + NAT + r * ROWB);
     }
     // One plain load for every lane, used only when the statistics go to LDS: a load under a
     // per-lane condition, or arithmetic on its result here, would make the wavefront wait
     // for it (and for the transfers issued before it) on the spot.
     const float* src = th < BT ? p.lse : p.delta;
-    st_reg = src[qrow0 + (long long)t * BT + (th & (BT - 1))];
+    const int row = half_row + t * BT + (th & (BT - 1));
+    st_reg = src[b * p.sq + (RAGGED ? min(row, p.sq - 1) : row)];
   };
-  auto store_stats = [&](int buf) {
+  auto store_stats = [&](int t, int buf) {
     unsigned char* base = lds + buf * DKV_HALF;
-    if (th < 2 * BT) reinterpret_cast<float*>(base + 2 * NAT)[th] = th < BT ? st_reg * LOG2E : -st_reg;
+    if (th < 2 * BT) {
+      float v = th < BT ? st_reg * LOG2E : -st_reg;
+      if (RAGGED && half_row + t * BT + (th & (BT - 1)) >= p.sq) v = th < BT ? INFINITY : 0.0f;
+      reinterpret_cast<float*>(base + 2 * NAT)[th] = v;
+    }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the transfers into this buffer have landed
   };
 
@@ -523,7 +525,7 @@ __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void at
   };
 
   int buf = 0;
-  store_stats(0);
+  store_stats(0, 0);
   // The K / V fragments came straight from memory: they are waited for here, once. Left
   // to the first MFMA that reads them, the wait would sit inside the loop, behind the
   // tile loads that every iteration has just issued.
@@ -534,7 +536,7 @@ __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void at
     const bool has_next = t + 1 < ntiles;
     if (has_next) issue_loads(t + 1, buf ^ 1);
     compute_tile(buf);
-    if (has_next) store_stats(buf ^ 1);
+    if (has_next) store_stats(t + 1, buf ^ 1);
     __syncthreads();
     buf ^= 1;
   }
@@ -551,7 +553,7 @@ __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void at
       }
   }
   __syncthreads();
-  if (qs == 1) return;
+  if (qs == 1 || !k_live) return;
   uint16_t* dk_out = reinterpret_cast<uint16_t*>(const_cast<char*>(chunk_entry(2, where.chunk)));
   uint16_t* dv_out = reinterpret_cast<uint16_t*>(const_cast<char*>(chunk_entry(3, where.chunk)));
 #pragma unroll
@@ -575,12 +577,8 @@ __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void at
 namespace jg {
 
 bool attn_mfma_bwd_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias) {
-  return dtype == JG_BF16 && !has_bias && d == D && sq > 0 && sk > 0 && sq % BR == 0 &&
-         sk % BR == 0 && sk % DKV_ROWS == 0 && batch > 0 && batch <= 65535;
-}
-
-size_t attn_mfma_bwd_workspace(long long batch, int sq, int) {
-  return (size_t)batch * sq * sizeof(float);
+  return dtype == JG_BF16 && !has_bias && d == D && sq > 0 && sk > 0 && sq <= ATTN_MAX_KEYS && sk <= ATTN_MAX_KEYS &&
+         batch > 0 && batch <= 65535;
 }
 
 // The ring backward over `nchunks` resident chunks: k[c], v[c] in, dk[c], dv[c] out, dq = the sum over
@@ -588,16 +586,7 @@ size_t attn_mfma_bwd_workspace(long long batch, int sq, int) {
 int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q,
                          const void* const* k, const void* const* v, int nchunks, const void* out, const float* lse,
                          long long batch, int sq, int sk, float scale, void* ws, hipStream_t s) {
-  if (nchunks < 1 || nchunks > MAX_CHUNKS)
-    JG_FAIL(JG_ERR_UNSUPPORTED, "jg_attn_bwd_chunks: 1 to %d chunks a call, got %d", MAX_CHUNKS, nchunks);
-  ChunkTable tab;
-  for (int c = 0; c < MAX_CHUNKS; ++c) {
-    const int u = c < nchunks ? c : 0;
-    tab.k[c] = static_cast<const uint16_t*>(k[u]);
-    tab.v[c] = static_cast<const uint16_t*>(v[u]);
-    tab.dk[c] = static_cast<uint16_t*>(dk[u]);
-    tab.dv[c] = static_cast<uint16_t*>(dv[u]);
-  }
+  const ChunkTable tab = chunk_table(k, v, dk, dv, nchunks);
   BwdArgs a;
   a.dout = static_cast<const uint16_t*>(dout);
   a.q = static_cast<const uint16_t*>(q);
@@ -612,25 +601,26 @@ int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
   a.scale = scale;
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e1 = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_bwd_dq_kernel),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, DQ_LDS);
-    hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_bwd_dkv_kernel),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, DKV_LDS);
-    if (e1 != hipSuccess || e2 != hipSuccess)
+    auto reserve = [](const void* f, int bytes) {
+      return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
+    };
+    if (!reserve(reinterpret_cast<const void*>(&attn_bwd_dq_kernel<false>), DQ_LDS) ||
+        !reserve(reinterpret_cast<const void*>(&attn_bwd_dq_kernel<true>), DQ_LDS) ||
+        !reserve(reinterpret_cast<const void*>(&attn_bwd_dkv_kernel<false>), DKV_LDS) ||
+        !reserve(reinterpret_cast<const void*>(&attn_bwd_dkv_kernel<true>), DKV_LDS))
       JG_FAIL(JG_ERR_LAUNCH, "jg_attn_bwd: cannot reserve LDS");
     attr_set = true;
   }
-  attn_bwd_dq_kernel<<<dim3((unsigned)(sq / BR), (unsigned)batch, 1), THREADS, DQ_LDS, s>>>(tab, a);
+  const bool ragged = sq % BR != 0 || sk % BR != 0 || sk % DKV_ROWS != 0;
+  const dim3 dq_grid((unsigned)cdiv(sq, BR), (unsigned)batch, 1);
+  const dim3 dkv_grid((unsigned)cdiv(sk, DKV_ROWS), (unsigned)batch, (unsigned)nchunks);
+  if (ragged) attn_bwd_dq_kernel<true><<<dq_grid, THREADS, DQ_LDS, s>>>(tab, a);
+  else attn_bwd_dq_kernel<false><<<dq_grid, THREADS, DQ_LDS, s>>>(tab, a);
   JG_CHECK_LAUNCH("jg_attn_bwd(dq)");
-  attn_bwd_dkv_kernel<<<dim3((unsigned)(sk / DKV_ROWS), (unsigned)batch, (unsigned)nchunks), DKV_THREADS, DKV_LDS, s>>>(tab, a);
+  if (ragged) attn_bwd_dkv_kernel<true><<<dkv_grid, DKV_THREADS, DKV_LDS, s>>>(tab, a);
+  else attn_bwd_dkv_kernel<false><<<dkv_grid, DKV_THREADS, DKV_LDS, s>>>(tab, a);
   JG_CHECK_LAUNCH("jg_attn_bwd(dkv)");
   return JG_OK;
-}
-
-int attn_mfma_bwd(void* dq, void* dk, void* dv, const void* dout, const void* q, const void* k,
-                  const void* v, const void* out, const float* lse, long long batch, int sq,
-                  int sk, float scale, void* ws, hipStream_t s) {
-  return attn_mfma_bwd_chunks(dq, &dk, &dv, dout, q, &k, &v, 1, out, lse, batch, sq, sk, scale, ws, s);
 }
 
 }  // namespace jg

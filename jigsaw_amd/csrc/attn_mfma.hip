@@ -41,9 +41,16 @@
 // Reference behaviour restated here:
 //   jigsaw/modules/attention/_functional/cores/math.py:69-78 (per-chunk core)
 //   jigsaw/modules/attention/_functional/forward.py:23-96    (merge per step)
-#include "jg_common.h"
+#include <initializer_list>
+
+#include "attn_chunks.h"
 
 namespace {
+
+using jg::BlockOf;
+using jg::ChunkTable;
+using jg::block_of;
+using jg::chunk_entry;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -71,6 +78,9 @@ constexpr int LDS_BYTES = NQ * QUARTER_BYTES;  // 131072
 // state, which a per-tile max would trigger in almost every tile of a 64-lane wavefront
 // (some query of 32 sees a new max), becomes the rare branch it is meant to be.
 constexpr float RESCALE_ABOVE = 8.0f;
+// The reference before the first tile: below any score, and finite, so that a key quarter without a single valid
+// key (RAGGED) ends with weight 0 instead of inf - inf.
+constexpr float NO_SCORE = -1.0e30f;
 constexpr int XO_FLOATS = 68 * 64;             // hand-over of one wavefront: 64 O registers + m, l per query block
 constexpr int STAGE_PITCH = 68;                // floats per query row of the staged result (64 + 4: 16-byte rows 4 banks apart)
 static_assert(4 * XO_FLOATS * 4 <= LDS_BYTES, "the hand-over slots reuse the tile buffers");
@@ -80,13 +90,12 @@ typedef short i16x4 __attribute__((ext_vector_type(4)));
 
 struct FwdArgs {
   const uint16_t* q;   // (batch, sq, 64)
-  const uint16_t* k;   // (batch, sk, 64)
-  const uint16_t* v;
   uint16_t* out;       // (batch, sq, 64) or NULL
   float* lse;          // (batch, sq) or NULL
   float* out_acc;      // (batch, sq, 64) fp32, merged in place, or NULL
   float* lse_acc;      // (batch, sq) fp32, merged in place, or NULL
-  int sq, sk;
+  int sq, sk;          // sk: keys per chunk
+  int nchunks;
   float scale;
 };
 
@@ -99,25 +108,13 @@ __device__ __forceinline__ void pair32(float v, float& a, float& b) {
   b = __uint_as_float(sw[1]);
 }
 
-// Workgroup -> (batch entry, row block). Consecutive workgroup ids go to the 8 XCDs in turn; each
-// XCD is given a contiguous range of (batch entry, block) pairs, so the workgroups that stream the
-// same K / V (or Q / dO) share one L2 instead of every L2 holding every head. Falls back to the
-// plain order when the count does not divide.
-struct BlockOf {
-  long long bh;
-  int blk;
-};
-__device__ __forceinline__ BlockOf block_of() {
-  const unsigned nblk = gridDim.x, total = gridDim.x * gridDim.y;
-  unsigned id = blockIdx.y * gridDim.x + blockIdx.x;
-  if ((total & 7u) == 0) id = (id & 7u) * (total >> 3) + (id >> 3);
-  BlockOf b;
-  b.bh = id / nblk;
-  b.blk = (int)(id % nblk);
-  return b;
-}
-
-__global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(FwdArgs p) {
+// RAGGED: sq or sk is no multiple of 128. The same kernel with the key rows of a transfer clamped to the chunk's
+// last one (three vector instructions per transfer), the scores of keys past the end set to -inf, query rows
+// clamped when read and dropped when written. 24 heads x 1000 queries x 2 chunks of 1000 keys: 93 us forward + backward
+// of the ring, against 832 us when the lengths were brought to multiples of 128 on the host (copies, a remainder of 104
+// keys on the one-thread-per-row kernel, two merges). The aligned kernel keeps its transfers free of vector instructions.
+template <bool RAGGED>
+__global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdArgs p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -126,8 +123,10 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(FwdArgs p) {
   const BlockOf where = block_of();
   const long long b = where.bh;
   const int q0 = where.blk * BM + qg * 64;
-  const int kquarter = p.sk >> 2;
-  const int ntiles = kquarter / BN;
+  // every chunk is cut in four key quarters (one per pair of wavefronts); a quarter's tiles of all chunks
+  // form one stream of ntiles tiles
+  const int qtiles = (p.sk + NQ * BN - 1) / (NQ * BN);
+  const int ntiles = qtiles * p.nchunks;
   const float c2 = p.scale * 1.4426950408889634f;  // scores are handled in base 2
 
   unsigned char* lds = smem + kq * QUARTER_BYTES;
@@ -136,7 +135,8 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(FwdArgs p) {
   bf16x8 qf[2][4];
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb) {
-    const uint16_t* qrow = p.q + (b * p.sq + q0 + qb * 32 + ln) * D + 8 * kg;
+    const int qi = q0 + qb * 32 + ln;
+    const uint16_t* qrow = p.q + (b * p.sq + (RAGGED ? min(qi, p.sq - 1) : qi)) * D + 8 * kg;
 #pragma unroll
     for (int c = 0; c < 4; ++c)
       qf[qb][c] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(qrow + 16 * c));
@@ -153,22 +153,46 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(FwdArgs p) {
   // every LDS read, which is how it orders LDS reads against transfers it knows about. The
   // kernel orders them itself: a buffer is read only after the wait + barrier that follows its
   // transfer, and refilled only after the barrier that follows its last read.)
-  const uint32_t dma_off = (uint32_t)((lane >> 3) * ROWB + (((lane & 7) ^ (lane >> 3)) << 4));
+  const uint32_t dma_swz = (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4);
+  const uint32_t dma_off = (uint32_t)((lane >> 3) * ROWB) + dma_swz;
   const int qg_u = __builtin_amdgcn_readfirstlane(qg), kq_u = __builtin_amdgcn_readfirstlane(kq);
-  const char* kdma = reinterpret_cast<const char*>(p.k + (b * p.sk + (long long)kq_u * kquarter) * D) + 16 * qg_u * ROWB;
-  const char* vdma = reinterpret_cast<const char*>(p.v + (b * p.sk + (long long)kq_u * kquarter) * D) + 16 * qg_u * ROWB;
   typedef __attribute__((address_space(3))) unsigned char* lds_bytes;
   const uint32_t lds_dma = (uint32_t)(uintptr_t)((lds_bytes)smem) + (uint32_t)(kq_u * QUARTER_BYTES + 16 * qg_u * ROWB);
-  auto dma_1k = [&](const char* src, uint32_t dst) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(dma_off), "s"(src), "s"(dst) : "m0");
+  auto dma_1k = [&](const char* src, uint32_t off, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(src), "s"(dst) : "m0");
   };
-  auto dma_tile = [&](int t, int buf) {
-    const long long off = (long long)t * KV_BYTES;
+  // the load cursor: tiles are requested in stream order, the last one again and again past the end
+  const long long chunk_off = 2 * (b * p.sk * (long long)D);  // bytes into a chunk
+  const int row_first = kq_u * qtiles * BN + 16 * qg_u;       // the wavefront's first row in the quarter
+  int ld_left = ntiles - 1, ld_tile = 0, ld_chunk = 0;
+  const char* kdma = chunk_entry(0, 0) + chunk_off;
+  const char* vdma = chunk_entry(1, 0) + chunk_off;
+  auto dma_tile = [&](int buf) {
     const uint32_t dst = lds_dma + (uint32_t)(buf * TILE_BYTES);
-    dma_1k(kdma + off, dst);
-    dma_1k(kdma + off + 8 * ROWB, dst + 8 * ROWB);
-    dma_1k(vdma + off, dst + KV_BYTES);
-    dma_1k(vdma + off + 8 * ROWB, dst + KV_BYTES + 8 * ROWB);
+    const int row = row_first + ld_tile * BN;
+    if (RAGGED) {
+      const uint32_t o0 = (uint32_t)min(row + (lane >> 3), p.sk - 1) * ROWB + dma_swz;
+      const uint32_t o1 = (uint32_t)min(row + 8 + (lane >> 3), p.sk - 1) * ROWB + dma_swz;
+      dma_1k(kdma, o0, dst);
+      dma_1k(kdma, o1, dst + 8 * ROWB);
+      dma_1k(vdma, o0, dst + KV_BYTES);
+      dma_1k(vdma, o1, dst + KV_BYTES + 8 * ROWB);
+    } else {
+      const long long off = (long long)row * ROWB;
+      dma_1k(kdma + off, dma_off, dst);
+      dma_1k(kdma + off + 8 * ROWB, dma_off, dst + 8 * ROWB);
+      dma_1k(vdma + off, dma_off, dst + KV_BYTES);
+      dma_1k(vdma + off + 8 * ROWB, dma_off, dst + KV_BYTES + 8 * ROWB);
+    }
+    if (ld_left > 0) {
+      --ld_left;
+      if (++ld_tile == qtiles) {
+        ld_tile = 0;
+        ++ld_chunk;
+        kdma = chunk_entry(0, ld_chunk) + chunk_off;
+        vdma = chunk_entry(1, ld_chunk) + chunk_off;
+      }
+    }
   };
   // per-lane constant parts of the fragment addresses
   //   K fragment c of key row ln: logical chunk 2 c + kg, stored at chunk (2 c + kg) ^ (ln % 8)
@@ -194,7 +218,7 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(FwdArgs p) {
     for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[qb][nb][i] = 0.0f;
-  float m[2] = {-INFINITY, -INFINITY};  // reference score of the lane's query (both lanes of a query agree)
+  float m[2] = {NO_SCORE, NO_SCORE};  // reference score of the lane's query (both lanes of a query agree)
   float l[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};  // running sums (two chains) of the probabilities of the lane's OWN 16 keys per block
 
   f32x16 s[2];       // scores of the two query blocks (half a step apart)
@@ -227,7 +251,7 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(FwdArgs p) {
   // Online softmax of the 32 x 32 score block of one query block, in two parts. First the
   // reference: when some lane of the wavefront sees a score more than RESCALE_ABOVE powers of
   // two over its reference (a rarely taken, wave-uniform branch; the first tile always takes
-  // it, its reference being -inf) the two lanes of each query agree on the tile's max, the
+  // it, its reference being NO_SCORE) the two lanes of each query agree on the tile's max, the
   // reference moves there and the state is rescaled. Then probabilities and partial row
   // sums: straight-line vector work that is interleaved with the matrix-core instructions
   // of the other query block.
@@ -296,10 +320,9 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(FwdArgs p) {
   // The transfer of tile t+3 is issued first, into the buffer tile t-1 has left. Past the
   // last tile the same instructions run on clamped tile indices and their results are
   // dropped, which keeps the loop body free of branches apart from the rare rescale.
-  const int last = ntiles - 1;
-  dma_tile(0, 0);
-  dma_tile(last < 1 ? last : 1, 1);
-  dma_tile(last < 2 ? last : 2, 2);
+  dma_tile(0);
+  dma_tile(1);
+  dma_tile(2);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
   load_kf(0);
@@ -322,7 +345,14 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(FwdArgs p) {
   // before the next half reads them (an MFMA chain of one wavefront shares the matrix core
   // with the other wavefront of the SIMD, so its last result arrives late); the two MFMAs in
   // front of the max are work for the matrix core while the vector unit runs the max tree.
+  // RAGGED: keys of the tile under the softmax from its first key to the chunk's end
+  int keys_left = p.sk - kq_u * qtiles * BN, soft_tile = 0;
   auto half = [&](int qa, int qo, auto&& after_scores, auto&& after_pv) {
+    if (RAGGED && keys_left < BN) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (8 * (i >> 2) + 4 * kg + (i & 3) >= keys_left) s[qa][i] = -INFINITY;
+    }
     score_one(qo, 0);
     score_one(qo, 1);
     JG_FENCE();
@@ -349,18 +379,25 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(FwdArgs p) {
     pin(pk[qa][0], pk[qa][1]);
     JG_FENCE();
   };
-  auto iteration = [&](int t, int cur, int nxt, int tgt) {
-    dma_tile(t + 3 < last ? t + 3 : last, tgt);
+  auto iteration = [&](int cur, int nxt, int tgt) {
+    dma_tile(tgt);
     // softmax of query block 0 (tile t) under: scores of block 1 (tile t), P V of block 1 (tile t-1)
     half(0, 1, [&]() { load_kf(nxt); }, [&]() { load_vf(cur); });
     // softmax of query block 1 (tile t) under: scores of block 0 (tile t+1), P V of block 0 (tile t)
     half(1, 0, [&]() {}, [&]() {});
+    if (RAGGED) {
+      keys_left -= BN;
+      if (++soft_tile == qtiles) {
+        soft_tile = 0;
+        keys_left += qtiles * BN;
+      }
+    }
     __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4): every transfer but this iteration's has landed
     __syncthreads();
   };
   // (unrolling over the four buffers would turn every LDS address into an immediate, but the
   // longer code ran no faster)
-  for (int t = 0; t < ntiles; ++t) iteration(t, t & 3, (t + 1) & 3, (t + 3) & 3);
+  for (int t = 0; t < ntiles; ++t) iteration(t & 3, (t + 1) & 3, (t + 3) & 3);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // the clamped transfers of the last iterations still target LDS
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt)
@@ -427,7 +464,7 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(FwdArgs p) {
       const float lse_j = (m[qb] * c2 + log2f(lt[qb])) * 0.6931471805599453f;  // natural log
       const int ql = qg * 64 + qb * 32 + ln;  // query inside the workgroup
       const long long qi = b * p.sq + where.blk * BM + ql;
-      if (kg == 0) {
+      if (kg == 0 && (!RAGGED || where.blk * BM + ql < p.sq)) {
         float w = 0.0f;
         if (p.out_acc != nullptr) {
           const float l_old = p.lse_acc[qi];
@@ -454,15 +491,17 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(FwdArgs p) {
   {
     const long long row0 = b * p.sq + (long long)where.blk * BM;
     f32x4 hv[4], acc[4];
+    const int rows_left = p.sq - where.blk * BM;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {  // piece e = tid + 512 i of the 128 x 16 pieces of 4 floats
       const int e = tid + THREADS * i;
       hv[i] = *reinterpret_cast<const f32x4*>(stage + (e >> 4) * STAGE_PITCH + 4 * (e & 15));
-      if (p.out_acc != nullptr) acc[i] = *reinterpret_cast<const f32x4*>(p.out_acc + row0 * D + 4 * (long long)e);
+      if (p.out_acc != nullptr && (!RAGGED || (e >> 4) < rows_left)) acc[i] = *reinterpret_cast<const f32x4*>(p.out_acc + row0 * D + 4 * (long long)e);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int e = tid + THREADS * i;
+      if (RAGGED && (e >> 4) >= rows_left) break;  // rows grow with i
       if (p.out != nullptr)
         *reinterpret_cast<bf16x4*>(p.out + row0 * D + 4 * (long long)e) = __builtin_convertvector(hv[i], bf16x4);
       if (p.out_acc != nullptr) {
@@ -483,33 +522,33 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(FwdArgs p) {
 namespace jg {
 
 bool attn_mfma_fwd_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias) {
-  return dtype == JG_BF16 && !has_bias && d == D && sq > 0 && sk > 0 && sq % BM == 0 &&
-         sk % (NQ * BN) == 0 && batch > 0 && batch <= 65535;
+  return dtype == JG_BF16 && !has_bias && d == D && sq > 0 && sk > 0 && sk <= ATTN_MAX_KEYS && batch > 0 && batch <= 65535;
 }
 
-int attn_mfma_fwd(void* out, float* lse, const void* q, const void* k, const void* v,
-                  long long batch, int sq, int sk, float scale, float* out_acc, float* lse_acc,
-                  hipStream_t s) {
+int attn_mfma_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v, int nchunks,
+                         long long batch, int sq, int sk, float scale, float* out_acc, float* lse_acc, hipStream_t s) {
   FwdArgs a;
   a.q = static_cast<const uint16_t*>(q);
-  a.k = static_cast<const uint16_t*>(k);
-  a.v = static_cast<const uint16_t*>(v);
   a.out = static_cast<uint16_t*>(out);
   a.lse = lse;
   a.out_acc = out_acc;
   a.lse_acc = lse_acc;
   a.sq = sq;
   a.sk = sk;
+  a.nchunks = nchunks;
   a.scale = scale;
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_fwd_mfma_kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);
-    if (e != hipSuccess) JG_FAIL(JG_ERR_LAUNCH, "jg_attn_fwd: cannot reserve %d bytes of LDS", LDS_BYTES);
+    for (const void* f : {reinterpret_cast<const void*>(&attn_fwd_mfma_kernel<false>),
+                          reinterpret_cast<const void*>(&attn_fwd_mfma_kernel<true>)})
+      if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES) != hipSuccess)
+        JG_FAIL(JG_ERR_LAUNCH, "jg_attn_fwd: cannot reserve %d bytes of LDS", LDS_BYTES);
     attr_set = true;
   }
-  dim3 grid((unsigned)(sq / BM), (unsigned)batch, 1);
-  attn_fwd_mfma_kernel<<<grid, THREADS, LDS_BYTES, s>>>(a);
+  const dim3 grid((unsigned)cdiv(sq, BM), (unsigned)batch, 1);
+  const ChunkTable tab = chunk_table(k, v, nullptr, nullptr, nchunks);
+  if (sq % BM == 0 && sk % (NQ * BN) == 0) attn_fwd_mfma_kernel<false><<<grid, THREADS, LDS_BYTES, s>>>(tab, a);
+  else attn_fwd_mfma_kernel<true><<<grid, THREADS, LDS_BYTES, s>>>(tab, a);
   JG_CHECK_LAUNCH("jg_attn_fwd(mfma)");
   return JG_OK;
 }

@@ -1,9 +1,21 @@
-// Blockwise (flash-style) attention of one K/V chunk on the bf16 / fp16 matrix cores for head
-// sizes 96 and 128, non-causal, no bias: forward (output + natural-log LSE) and backward
-// from a given (global) output and LSE. Same arithmetic as the head-size-64 kernels,
-// written for clarity rather than hand-scheduled: tiles of 32 keys (forward, dQ) or 32
-// queries (dK/dV) pass through a double-buffered LDS stage, fetched to registers one tile
-// ahead.
+// Blockwise (flash-style) attention over the K/V chunks of a ring on the bf16 / fp16 matrix cores for
+// head sizes up to 128 (multiples of 8), any lengths, non-causal, no bias: forward (output +
+// natural-log LSE) and backward from a given (global) output and LSE. Same arithmetic as the
+// bf16 kernels of head size 64, written for clarity rather than hand-scheduled: tiles of 32 keys
+// (forward, dQ) or 32 queries (dK/dV) pass through a double-buffered LDS stage, fetched to
+// registers one tile ahead.
+//
+//   widths         kernels of 32, 64, 96 and 128 columns (D); a smaller head is staged with zeros in
+//                  the columns it does not have. Rows past the end of a tensor are staged as zeros
+//                  too; keys past the end get the score -inf, queries past the end the lse +inf.
+//   groups         a workgroup is KS groups of four wavefronts. A group walks every KS-th tile of
+//                  the streamed side with a stage of its own, and the groups' sums are combined
+//                  through LDS at the end: where a launch has fewer workgroups than the chip has
+//                  CUs, more wavefronts share the rows of one (see split_of on the host side).
+//
+// Forward + backward of a ring, before (lengths and head size padded on the host, one launch and one merge per
+// chunk) and now: 4 heads x 128 x 2 chunks of 128 keys, head size 32: 402 -> 48 us (host time); 12 heads x 869 x 869,
+// head size 96, fp16: 528 -> 99 us; 16 heads x 2424 x 2424, head size 32, fp16: 568 -> 225 us.
 //
 //   forward / dQ   lane = query. S^T = K Q^T (A = K rows from LDS, B = Q rows kept in
 //                  registers), so the running max / sum, lse and delta of a query are
@@ -20,9 +32,16 @@
 // Reference behaviour restated here:
 //   jigsaw/modules/attention/_functional/cores/math.py:69-78   (forward)
 //   jigsaw/modules/attention/_functional/cores/math.py:125-149 (backward)
-#include "jg_common.h"
+#include <type_traits>
+
+#include "attn_chunks.h"
 
 namespace {
+
+using jg::BlockOf;
+using jg::ChunkTable;
+using jg::block_of;
+using jg::chunk_entry;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -34,10 +53,11 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int WAVES = 4, THREADS = WAVES * 64;
-constexpr int BQ = 32 * WAVES;  // rows (queries or keys) of a workgroup, 32 per wavefront
+constexpr int WAVES = 4, GROUP = WAVES * 64;  // wavefronts and threads of a group
+constexpr int BQ = 32 * WAVES;  // rows (queries or keys) of a workgroup, 32 per wavefront of a group
 constexpr int BT = 32;          // rows of a streamed tile
 constexpr float LOG2E = 1.4426950408889634f;
+constexpr float NO_SCORE = -1.0e30f;  // running maximum before the first key: finite, so that a group without a key weighs 0
 
 template <int D>
 struct Geo {
@@ -46,7 +66,7 @@ struct Geo {
   static constexpr int TP = BT * 2 + 16;  // bytes per row of a transposed tile (D rows of 32)
   static constexpr int ROWMAJ = BT * RP, TRANS = D * TP;
   static constexpr int CHUNKS = BT * D / 8;  // 16-byte pieces of a tile
-  static constexpr int PER = (CHUNKS + THREADS - 1) / THREADS;
+  static constexpr int PER = (CHUNKS + GROUP - 1) / GROUP;
 };
 
 // Column of a transposed tile that holds tile row x: inside a group of 16 rows the order is the
@@ -58,20 +78,31 @@ struct TileRegs {
   u32x4 v[Geo<D>::PER];
 };
 
-// 32 rows x D of a row-major (row stride D) bf16 matrix to registers
+// 32 rows of a row-major matrix of row length d <= D to registers; rows from `rows` on and columns from d on are
+// zero. tid: thread of the group.
 template <int D>
-__device__ __forceinline__ void tile_fetch(TileRegs<D>& r, const uint16_t* src) {
+__device__ __forceinline__ void tile_fetch(TileRegs<D>& r, const uint16_t* src, int tid, int rows, int d) {
+  if (rows >= BT && d == D) {  // wave-uniform
+#pragma unroll
+    for (int i = 0; i < Geo<D>::PER; ++i) {
+      const int c = tid + i * GROUP;
+      if (c < Geo<D>::CHUNKS) r.v[i] = *reinterpret_cast<const u32x4*>(src + c * 8);  // rows are contiguous: chunk c = 8 elements at c*8
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < Geo<D>::PER; ++i) {
-    const int c = threadIdx.x + i * THREADS;
-    if (c < Geo<D>::CHUNKS) r.v[i] = *reinterpret_cast<const u32x4*>(src + c * 8);  // rows are contiguous: chunk c = 8 elements at c*8
+    const int c = tid + i * GROUP;
+    const int row = c / (D / 8), col = (c % (D / 8)) * 8;
+    r.v[i] = u32x4{0u, 0u, 0u, 0u};
+    if (c < Geo<D>::CHUNKS && row < rows && col < d) r.v[i] = *reinterpret_cast<const u32x4*>(src + row * d + col);
   }
 }
 template <int D>
-__device__ __forceinline__ void tile_store_rows(const TileRegs<D>& r, unsigned char* dst) {
+__device__ __forceinline__ void tile_store_rows(const TileRegs<D>& r, unsigned char* dst, int tid) {
 #pragma unroll
   for (int i = 0; i < Geo<D>::PER; ++i) {
-    const int c = threadIdx.x + i * THREADS;
+    const int c = tid + i * GROUP;
     if (c < Geo<D>::CHUNKS) {
       const int row = c / (D / 8), col8 = c % (D / 8);
       *reinterpret_cast<u32x4*>(dst + row * Geo<D>::RP + col8 * 16) = r.v[i];
@@ -85,17 +116,23 @@ struct TransRegs {
   uint32_t w[8];
 };
 template <int D>
-__device__ __forceinline__ void trans_fetch(TransRegs<D>& r, const uint16_t* src) {
-  if (threadIdx.x < 4 * (D / 2)) {
-    const int g8 = threadIdx.x / (D / 2), cp = threadIdx.x % (D / 2);
+__device__ __forceinline__ void trans_fetch(TransRegs<D>& r, const uint16_t* src, int tid, int rows, int d) {
+  if (tid < 4 * (D / 2)) {
+    const int g8 = tid / (D / 2), cp = tid % (D / 2);
+    if (rows >= BT && d == D) {  // wave-uniform
 #pragma unroll
-    for (int i = 0; i < 8; ++i) r.w[i] = *reinterpret_cast<const uint32_t*>(src + (g8 * 8 + i) * D + 2 * cp);
+      for (int i = 0; i < 8; ++i) r.w[i] = *reinterpret_cast<const uint32_t*>(src + (g8 * 8 + i) * D + 2 * cp);
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      r.w[i] = (g8 * 8 + i < rows && 2 * cp < d) ? *reinterpret_cast<const uint32_t*>(src + (g8 * 8 + i) * d + 2 * cp) : 0u;
   }
 }
 template <int D>
-__device__ __forceinline__ void trans_store(const TransRegs<D>& r, unsigned char* dst) {
-  if (threadIdx.x < 4 * (D / 2)) {
-    const int g8 = threadIdx.x / (D / 2), cp = threadIdx.x % (D / 2);
+__device__ __forceinline__ void trans_store(const TransRegs<D>& r, unsigned char* dst, int tid) {
+  if (tid < 4 * (D / 2)) {
+    const int g8 = tid / (D / 2), cp = tid % (D / 2);
     // rows 8*g8 .. 8*g8+7 of the tile: the first four land at the place of row 8*g8, the last four 8 places on
     const int pos_lo = (g8 >> 1) * 16 + (g8 & 1) * 4, pos_hi = pos_lo + 8;
 #pragma unroll
@@ -175,27 +212,34 @@ __device__ __forceinline__ u32x2 pack4(float a, float b, float c, float d) {
   return r;
 }
 
-// Workgroup -> (batch entry, row block). Consecutive workgroup ids go to the 8 XCDs in turn; each
-// XCD is given a contiguous range of (batch entry, block) pairs, so the workgroups that stream the
-// same K / V (or Q / dO) share one L2. Falls back to the plain order when the count does not divide.
-struct BlockOf {
-  long long bh;
-  int blk;
-};
-__device__ __forceinline__ BlockOf block_of() {
-  const unsigned nblk = gridDim.x, total = gridDim.x * gridDim.y;
-  unsigned id = blockIdx.y * gridDim.x + blockIdx.x;
-  if ((total & 7u) == 0) id = (id & 7u) * (total >> 3) + (id >> 3);
-  BlockOf b;
-  b.bh = id / nblk;
-  b.blk = (int)(id % nblk);
-  return b;
+// 16-byte piece `col` / 8 of a row in memory, zero past the head's columns
+template <int D, bool F16>
+__device__ __forceinline__ typename Half<F16>::x8 row_frag(const uint16_t* row, int col, int d) {
+  u32x4 v = {0u, 0u, 0u, 0u};
+  if (col < d) v = *reinterpret_cast<const u32x4*>(row + col);
+  return __builtin_bit_cast(typename Half<F16>::x8, v);
 }
+
+// Which tile of which chunk a group takes next: tiles ks, ks + KS, ... of every chunk in turn. Every group makes
+// `steps` steps a chunk; in a step past the chunk's end rows_left is <= 0.
+template <int KS>
+struct Stream {
+  int steps, rows, tile, step, chunk;
+  __device__ Stream(int rows_, int ks) : steps((rows_ + BT * KS - 1) / (BT * KS)), rows(rows_), tile(ks), step(0), chunk(0) {}
+  __device__ __forceinline__ int first_row() const { return tile * BT; }
+  __device__ __forceinline__ int rows_left() const { return rows - tile * BT; }
+  __device__ __forceinline__ void next() {
+    tile += KS;
+    if (++step == steps) {
+      step = 0;
+      tile -= steps * KS;
+      ++chunk;
+    }
+  }
+};
 
 struct Args {
   const uint16_t* q;
-  const uint16_t* k;
-  const uint16_t* v;
   const uint16_t* out;   // backward: the global output
   const uint16_t* dout;  // backward
   const float* lse_in;   // backward: the global lse
@@ -205,45 +249,58 @@ struct Args {
   float* out_acc;        // forward: fp32 (batch, sq, d) accumulator of the ring, merged in place, or NULL
   float* lse_acc;        // forward: fp32 (batch, sq), merged in place, or NULL
   uint16_t* dq;
-  uint16_t* dk;
-  uint16_t* dv;
-  int sq, sk;
+  int sq, sk;            // sk: keys per chunk
+  int d;                 // columns of a head, <= D and a multiple of 8
+  int nchunks;
   float scale;
 };
 
 // ------------------------------------------------------------------- forward
-template <int D, bool F16>
-__global__ __launch_bounds__(THREADS) void attn_wide_fwd_kernel(Args p) {
+template <int D, bool F16, int KS>
+__global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, Args p) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
   constexpr int BUF = G::ROWMAJ + G::TRANS;  // K rows, then V^T
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2 * BUF];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x % GROUP, ks = threadIdx.x / GROUP;
+  const int lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kg = lane >> 5;
   const BlockOf wg = block_of();
   const long long bh = wg.bh;
   const int qi = wg.blk * BQ + wave * 32 + ln;
-  const uint16_t* qrow = p.q + (bh * p.sq + qi) * D;
-  const uint16_t* kb = p.k + bh * p.sk * D;
-  const uint16_t* vb = p.v + bh * p.sk * D;
+  const bool live = qi < p.sq;
+  const uint16_t* qrow = p.q + (bh * p.sq + (live ? qi : p.sq - 1)) * p.d;
+  const long long chunk_off = bh * p.sk * p.d;
   const float c2 = p.scale * LOG2E;
+  unsigned char* lds = smem + ks * 2 * BUF;
 
   X8 qf[G::C16];
 #pragma unroll
-  for (int c = 0; c < G::C16; ++c) qf[c] = frag<F16>(reinterpret_cast<const unsigned char*>(qrow + 16 * c + 8 * kg));
+  for (int c = 0; c < G::C16; ++c) qf[c] = row_frag<D, F16>(qrow, 16 * c + 8 * kg, p.d);
 
   f32x16 o[G::NB];
 #pragma unroll
   for (int nb = 0; nb < G::NB; ++nb) o[nb] = zero16();
-  float m = -INFINITY, l = 0.0f;
+  float m = NO_SCORE, l = 0.0f;
 
   TileRegs<D> rk;
   TransRegs<D> rv;
-  const int ntiles = p.sk / BT;
-  tile_fetch<D>(rk, kb);
-  trans_fetch<D>(rv, vb);
-  tile_store_rows<D>(rk, smem);
-  trans_store<D>(rv, smem + G::ROWMAJ);
+  Stream<KS> load(p.sk, ks), soft(p.sk, ks);
+  const int ntiles = load.steps * p.nchunks;
+  auto fetch = [&]() {
+    const uint16_t* kb = reinterpret_cast<const uint16_t*>(chunk_entry(0, load.chunk)) + chunk_off;
+    const uint16_t* vb = reinterpret_cast<const uint16_t*>(chunk_entry(1, load.chunk)) + chunk_off;
+    const long long at = (long long)load.first_row() * p.d;
+    tile_fetch<D>(rk, kb + at, tid, load.rows_left(), p.d);
+    trans_fetch<D>(rv, vb + at, tid, load.rows_left(), p.d);
+    load.next();
+  };
+  auto store = [&](int buf) {
+    tile_store_rows<D>(rk, lds + buf * BUF, tid);
+    trans_store<D>(rv, lds + buf * BUF + G::ROWMAJ, tid);
+  };
+  fetch();
+  store(0);
   // The fragments that came straight from memory are waited for here, once. Left to the first matrix
   // instruction that reads them, the wait sits inside the loop, behind the tile loads every iteration has
   // just issued, and counts those too: each iteration then waited for its own prefetch.
@@ -251,17 +308,20 @@ __global__ __launch_bounds__(THREADS) void attn_wide_fwd_kernel(Args p) {
   for (int c = 0; c < G::C16; ++c) asm volatile("" : "+v"(qf[c]));
   __syncthreads();
   for (int t = 0; t < ntiles; ++t) {
-    const unsigned char* kt = smem + (t & 1) * BUF;
+    const unsigned char* kt = lds + (t & 1) * BUF;
     const unsigned char* vt = kt + G::ROWMAJ;
-    if (t + 1 < ntiles) {
-      tile_fetch<D>(rk, kb + (long long)(t + 1) * BT * D);
-      trans_fetch<D>(rv, vb + (long long)(t + 1) * BT * D);
-    }
+    if (t + 1 < ntiles) fetch();
     // S^T: lane = query ln, register i = key 8*(i/4) + 4*kg + i%4 of the tile
     f32x16 s = zero16();
 #pragma unroll
     for (int c = 0; c < G::C16; ++c)
       s = Half<F16>::mma(frag<F16>(kt + ln * G::RP + (16 * c + 8 * kg) * 2), qf[c], s);
+    if (soft.rows_left() < BT) {  // wave-uniform
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (8 * (i >> 2) + 4 * kg + (i & 3) >= soft.rows_left()) s[i] = -INFINITY;
+    }
+    soft.next();
     float mx = s[0];
 #pragma unroll
     for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
@@ -269,7 +329,7 @@ __global__ __launch_bounds__(THREADS) void attn_wide_fwd_kernel(Args p) {
     const float mn = fmaxf(m, mx);
     // the maximum settles after a few tiles: rescale only when some query of the wavefront saw a larger score
     if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {
-      const float alpha = __builtin_amdgcn_exp2f((m - mn) * c2);  // first tile: exp2(-inf) = 0
+      const float alpha = __builtin_amdgcn_exp2f((m - mn) * c2);  // first tile: 0
       l *= alpha;
 #pragma unroll
       for (int nb = 0; nb < G::NB; ++nb)
@@ -293,15 +353,44 @@ __global__ __launch_bounds__(THREADS) void attn_wide_fwd_kernel(Args p) {
         o[nb] = Half<F16>::mma(frag<F16>(vt + (nb * 32 + ln) * G::TP + (16 * ks + 8 * kg) * 2), pf,
                                                         o[nb]);
     }
-    if (t + 1 < ntiles) {
-      unsigned char* nk = smem + ((t + 1) & 1) * BUF;
-      tile_store_rows<D>(rk, nk);
-      trans_store<D>(rv, nk + G::ROWMAJ);
-    }
+    if (t + 1 < ntiles) store((t + 1) & 1);
     __syncthreads();
   }
   // the two lanes of a query saw the same maxima; their sums cover disjoint keys
   l += __shfl_xor(l, 32, 64);
+  if constexpr (KS > 1) {
+    // the groups hand over to the one below them, halving their number each time
+    constexpr int XO = (16 * G::NB + 2) * 64;  // floats of a wavefront
+    static_assert(KS / 2 * WAVES * XO * 4 <= KS * 2 * BUF, "the hand-over reuses the stages");
+    float* xo = reinterpret_cast<float*>(smem) + ((ks % (KS / 2)) * WAVES + wave) * XO + lane;
+#pragma unroll
+    for (int half = KS / 2; half >= 1; half >>= 1) {
+      if (ks >= half && ks < 2 * half) {
+        float* to = reinterpret_cast<float*>(smem) + ((ks - half) * WAVES + wave) * XO + lane;
+#pragma unroll
+        for (int nb = 0; nb < G::NB; ++nb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) to[(nb * 16 + i) * 64] = o[nb][i];
+        to[16 * G::NB * 64] = m;
+        to[(16 * G::NB + 1) * 64] = l;
+      }
+      __syncthreads();
+      if (ks < half) {
+        const float m1 = xo[16 * G::NB * 64], l1 = xo[(16 * G::NB + 1) * 64];
+        const float mn = fmaxf(m, m1);
+        const float a0 = __builtin_amdgcn_exp2f((m - mn) * c2), a1 = __builtin_amdgcn_exp2f((m1 - mn) * c2);
+        l = l * a0 + l1 * a1;
+        m = mn;
+#pragma unroll
+        for (int nb = 0; nb < G::NB; ++nb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[nb][i] = o[nb][i] * a0 + xo[(nb * 16 + i) * 64] * a1;
+      }
+      __syncthreads();
+    }
+    if (ks != 0) return;
+  }
+  if (!live) return;
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
   const float lse_j = l > 0.0f ? m * p.scale + __logf(l) : -INFINITY;
   const long long row = bh * p.sq + qi;
@@ -320,10 +409,11 @@ __global__ __launch_bounds__(THREADS) void attn_wide_fwd_kernel(Args p) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int dv = nb * 32 + 8 * j + 4 * kg;
+      if (dv >= p.d) continue;
       const u32x2 h = pack4<F16>(o[nb][4 * j] * inv, o[nb][4 * j + 1] * inv, o[nb][4 * j + 2] * inv, o[nb][4 * j + 3] * inv);
-      if (p.o != nullptr) *reinterpret_cast<u32x2*>(p.o + row * D + dv) = h;
+      if (p.o != nullptr) *reinterpret_cast<u32x2*>(p.o + row * p.d + dv) = h;
       if (p.out_acc != nullptr) {
-        f32x4* dst = reinterpret_cast<f32x4*>(p.out_acc + row * D + dv);
+        f32x4* dst = reinterpret_cast<f32x4*>(p.out_acc + row * p.d + dv);
         f32x4 a = *dst;
         float h0, h1, h2, h3;
         Half<F16>::unpair(h.x, h0, h1);
@@ -338,35 +428,37 @@ __global__ __launch_bounds__(THREADS) void attn_wide_fwd_kernel(Args p) {
 }
 
 // ------------------------------------------------------------------- dQ (and delta)
-template <int D, bool F16>
-__global__ __launch_bounds__(THREADS) void attn_wide_dq_kernel(Args p) {
+template <int D, bool F16, int KS>
+__global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Args p) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
   constexpr int BUF = 2 * G::ROWMAJ + G::TRANS;  // K rows, V rows, K^T
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int tid = threadIdx.x % GROUP, ks = threadIdx.x / GROUP;
+  const int lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kg = lane >> 5;
   const BlockOf wg = block_of();
   const long long bh = wg.bh;
-  const int qi = wg.blk * BQ + wave * 32 + ln;
-  const long long qoff = (bh * p.sq + qi) * D;
-  const uint16_t* kb = p.k + bh * p.sk * D;
-  const uint16_t* vb = p.v + bh * p.sk * D;
+  const bool live = wg.blk * BQ + wave * 32 + ln < p.sq;
+  const int qi = live ? wg.blk * BQ + wave * 32 + ln : p.sq - 1;
+  const long long qoff = (bh * p.sq + qi) * p.d;
+  const long long chunk_off = bh * p.sk * p.d;
   const float c2 = p.scale * LOG2E;
+  unsigned char* lds = smem + ks * 2 * BUF;
 
   X8 qf[G::C16], dof[G::C16];
   float dl = 0.0f;
 #pragma unroll
   for (int c = 0; c < G::C16; ++c) {
-    qf[c] = frag<F16>(reinterpret_cast<const unsigned char*>(p.q + qoff + 16 * c + 8 * kg));
-    dof[c] = frag<F16>(reinterpret_cast<const unsigned char*>(p.dout + qoff + 16 * c + 8 * kg));
-    const X8 of = frag<F16>(reinterpret_cast<const unsigned char*>(p.out + qoff + 16 * c + 8 * kg));
+    qf[c] = row_frag<D, F16>(p.q + qoff, 16 * c + 8 * kg, p.d);
+    dof[c] = row_frag<D, F16>(p.dout + qoff, 16 * c + 8 * kg, p.d);
+    const X8 of = row_frag<D, F16>(p.out + qoff, 16 * c + 8 * kg, p.d);
 #pragma unroll
     for (int j = 0; j < 8; ++j) dl += (float)dof[c][j] * (float)of[j];
   }
   // delta = rowsum(dO o O): the two lanes of a query hold disjoint halves of the row
   const float delta = dl + __shfl_xor(dl, 32, 64);
-  if (kg == 0) p.delta[bh * p.sq + qi] = delta;
+  if (kg == 0 && ks == 0 && live) p.delta[bh * p.sq + qi] = delta;
   const float lse2 = p.lse_in[bh * p.sq + qi] * LOG2E;
 
   f32x16 dq[G::NB];
@@ -375,34 +467,46 @@ __global__ __launch_bounds__(THREADS) void attn_wide_dq_kernel(Args p) {
 
   TileRegs<D> rk, rv;
   TransRegs<D> rkt;
-  const int ntiles = p.sk / BT;
-  tile_fetch<D>(rk, kb);
-  tile_fetch<D>(rv, vb);
-  trans_fetch<D>(rkt, kb);
-  tile_store_rows<D>(rk, smem);
-  tile_store_rows<D>(rv, smem + G::ROWMAJ);
-  trans_store<D>(rkt, smem + 2 * G::ROWMAJ);
-  // The fragments that came straight from memory are waited for here, once. Left to the first matrix
-  // instruction that reads them, the wait sits inside the loop, behind the tile loads every iteration has
-  // just issued, and counts those too: each iteration then waited for its own prefetch.
+  Stream<KS> load(p.sk, ks), soft(p.sk, ks);
+  const int ntiles = load.steps * p.nchunks;
+  auto fetch = [&]() {
+    const long long at = chunk_off + (long long)load.first_row() * p.d;
+    const uint16_t* kb = reinterpret_cast<const uint16_t*>(chunk_entry(0, load.chunk)) + at;
+    const uint16_t* vb = reinterpret_cast<const uint16_t*>(chunk_entry(1, load.chunk)) + at;
+    tile_fetch<D>(rk, kb, tid, load.rows_left(), p.d);
+    tile_fetch<D>(rv, vb, tid, load.rows_left(), p.d);
+    trans_fetch<D>(rkt, kb, tid, load.rows_left(), p.d);
+    load.next();
+  };
+  auto store = [&](int buf) {
+    unsigned char* at = lds + buf * BUF;
+    tile_store_rows<D>(rk, at, tid);
+    tile_store_rows<D>(rv, at + G::ROWMAJ, tid);
+    trans_store<D>(rkt, at + 2 * G::ROWMAJ, tid);
+  };
+  fetch();
+  store(0);
+  // waited for once, here (see the forward kernel)
 #pragma unroll
   for (int c = 0; c < G::C16; ++c) asm volatile("" : "+v"(qf[c]), "+v"(dof[c]));
   __syncthreads();
   for (int t = 0; t < ntiles; ++t) {
-    const unsigned char* kt = smem + (t & 1) * BUF;
+    const unsigned char* kt = lds + (t & 1) * BUF;
     const unsigned char* vt = kt + G::ROWMAJ;
     const unsigned char* ktt = kt + 2 * G::ROWMAJ;
-    if (t + 1 < ntiles) {
-      tile_fetch<D>(rk, kb + (long long)(t + 1) * BT * D);
-      tile_fetch<D>(rv, vb + (long long)(t + 1) * BT * D);
-      trans_fetch<D>(rkt, kb + (long long)(t + 1) * BT * D);
-    }
+    if (t + 1 < ntiles) fetch();
     f32x16 s = zero16(), dp = zero16();
 #pragma unroll
     for (int c = 0; c < G::C16; ++c) {
       s = Half<F16>::mma(frag<F16>(kt + ln * G::RP + (16 * c + 8 * kg) * 2), qf[c], s);
       dp = Half<F16>::mma(frag<F16>(vt + ln * G::RP + (16 * c + 8 * kg) * 2), dof[c], dp);
     }
+    if (soft.rows_left() < BT) {  // wave-uniform
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (8 * (i >> 2) + 4 * kg + (i & 3) >= soft.rows_left()) s[i] = -INFINITY;
+    }
+    soft.next();
     float ds[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) ds[i] = __builtin_amdgcn_exp2f(s[i] * c2 - lse2) * (dp[i] - delta);
@@ -414,55 +518,75 @@ __global__ __launch_bounds__(THREADS) void attn_wide_dq_kernel(Args p) {
         dq[nb] = Half<F16>::mma(frag<F16>(ktt + (nb * 32 + ln) * G::TP + (16 * ks + 8 * kg) * 2),
                                                          dsf, dq[nb]);
     }
-    if (t + 1 < ntiles) {
-      unsigned char* nk = smem + ((t + 1) & 1) * BUF;
-      tile_store_rows<D>(rk, nk);
-      tile_store_rows<D>(rv, nk + G::ROWMAJ);
-      trans_store<D>(rkt, nk + 2 * G::ROWMAJ);
-    }
+    if (t + 1 < ntiles) store((t + 1) & 1);
     __syncthreads();
   }
+  if constexpr (KS > 1) {
+    static_assert(KS == 2 && WAVES * 16 * G::NB * 64 * 4 <= KS * 2 * BUF, "the hand-over reuses the stages");
+    float* xo = reinterpret_cast<float*>(smem) + wave * 16 * G::NB * 64 + lane;
+    if (ks == 1) {
+#pragma unroll
+      for (int nb = 0; nb < G::NB; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) xo[(nb * 16 + i) * 64] = dq[nb][i];
+    }
+    __syncthreads();
+    if (ks == 1) return;
+#pragma unroll
+    for (int nb = 0; nb < G::NB; ++nb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dq[nb][i] += xo[(nb * 16 + i) * 64];
+  }
+  if (!live) return;
   uint16_t* row = p.dq + qoff;
 #pragma unroll
   for (int nb = 0; nb < G::NB; ++nb)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      *reinterpret_cast<u32x2*>(row + nb * 32 + 8 * j + 4 * kg) =
-          pack4<F16>(dq[nb][4 * j] * p.scale, dq[nb][4 * j + 1] * p.scale, dq[nb][4 * j + 2] * p.scale,
-                dq[nb][4 * j + 3] * p.scale);
+    for (int j = 0; j < 4; ++j) {
+      const int col = nb * 32 + 8 * j + 4 * kg;
+      if (col < p.d)
+        *reinterpret_cast<u32x2*>(row + col) = pack4<F16>(dq[nb][4 * j] * p.scale, dq[nb][4 * j + 1] * p.scale,
+                                                          dq[nb][4 * j + 2] * p.scale, dq[nb][4 * j + 3] * p.scale);
+    }
 }
 
 // ------------------------------------------------------------------- dK, dV
 // MODE 0 forms dK and dV in one pass (two d x 32 accumulators a wavefront). That fits two workgroups
 // per CU in 256 registers a lane at head size 96 but not at 128 (it would spill, and ran 1.3x slower
-// that way), so head size 128 runs the kernel twice: MODE 1 forms dV only (from P), MODE 2 dK only
+// that way), so head sizes above 96 run the kernel twice: MODE 1 forms dV only (from P), MODE 2 dK only
 // (from dS), each with one accumulator and two workgroups per CU; the scores are computed in both.
 // A launch with no more workgroups than CUs gains nothing from that and keeps the single pass.
-template <int D, bool F16, int MODE>
-__global__ __launch_bounds__(THREADS, (D <= 96 || MODE != 0) ? 2 : 1) void attn_wide_dkv_kernel(Args p) {
+template <int D, bool F16, int MODE, int KS>
+__global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 : 1) void attn_wide_dkv_kernel(ChunkTable, Args p) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
   constexpr bool DV = MODE != 2, DK = MODE != 1;
   constexpr int STATS = 2 * BT * 4;                           // lse * log2(e) and delta of the tile's queries
   constexpr int BUF = 2 * G::ROWMAJ + 2 * G::TRANS + STATS;   // Q rows, dO rows, Q^T, dO^T, stats
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int tid = threadIdx.x % GROUP, ks = threadIdx.x / GROUP;
+  const int lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kg = lane >> 5;
   const BlockOf wg = block_of();
   const long long bh = wg.bh;
-  const int ki = wg.blk * BQ + wave * 32 + ln;
-  const long long koff = (bh * p.sk + ki) * D;
-  const uint16_t* qb = p.q + bh * p.sq * D;
-  const uint16_t* gb = p.dout + bh * p.sq * D;
+  const bool live = wg.blk * BQ + wave * 32 + ln < p.sk;
+  const long long koff = (bh * p.sk + (live ? wg.blk * BQ + wave * 32 + ln : p.sk - 1)) * p.d;
+  const uint16_t* qb = p.q + bh * p.sq * p.d;
+  const uint16_t* gb = p.dout + bh * p.sq * p.d;
   const float* lb = p.lse_in + bh * p.sq;
   const float* db = p.delta + bh * p.sq;
   const float c2 = p.scale * LOG2E;
+  unsigned char* lds = smem + ks * 2 * BUF;
 
   X8 kf[G::C16], vf[DK ? G::C16 : 1];
+  {
+    const uint16_t* krow = reinterpret_cast<const uint16_t*>(chunk_entry(0, wg.chunk)) + koff;
+    const uint16_t* vrow = reinterpret_cast<const uint16_t*>(chunk_entry(1, wg.chunk)) + koff;
 #pragma unroll
-  for (int c = 0; c < G::C16; ++c) {
-    kf[c] = frag<F16>(reinterpret_cast<const unsigned char*>(p.k + koff + 16 * c + 8 * kg));
-    if (DK) vf[c] = frag<F16>(reinterpret_cast<const unsigned char*>(p.v + koff + 16 * c + 8 * kg));
+    for (int c = 0; c < G::C16; ++c) {
+      kf[c] = row_frag<D, F16>(krow, 16 * c + 8 * kg, p.d);
+      if (DK) vf[c] = row_frag<D, F16>(vrow, 16 * c + 8 * kg, p.d);
+    }
   }
   f32x16 dk[DK ? G::NB : 1], dv[DV ? G::NB : 1];
 #pragma unroll
@@ -473,32 +597,39 @@ __global__ __launch_bounds__(THREADS, (D <= 96 || MODE != 0) ? 2 : 1) void attn_
 
   TileRegs<D> rq, rg;        // Q rows (scores); dO rows (dP: dK only)
   TransRegs<D> rqt, rgt;     // Q^T (dK only); dO^T (dV only)
-  float st = 0.0f;  // one statistic per thread of the first wavefront: lse2 (lanes 0-31) or delta (32-63)
-  const int ntiles = p.sq / BT;
-  auto fetch = [&](int t) {
-    tile_fetch<D>(rq, qb + (long long)t * BT * D);
-    if (DK) tile_fetch<D>(rg, gb + (long long)t * BT * D);
-    if (DK) trans_fetch<D>(rqt, qb + (long long)t * BT * D);
-    if (DV) trans_fetch<D>(rgt, gb + (long long)t * BT * D);
-    if (threadIdx.x < 2 * BT) {
-      const float* src = threadIdx.x < BT ? lb : db;  // every lane loads; the factor is applied when stored
-      st = src[t * BT + (threadIdx.x & (BT - 1))];
+  float st = 0.0f;  // one statistic per thread of the group's first wavefront: lse2 (lanes 0-31) or delta (32-63)
+  int st_rows = 0;  // rows of the tile it belongs to
+  Stream<KS> load(p.sq, ks);
+  const int ntiles = load.steps;
+  auto fetch = [&]() {
+    const long long at = (long long)load.first_row() * p.d;
+    const int rows = load.rows_left();
+    tile_fetch<D>(rq, qb + at, tid, rows, p.d);
+    if (DK) tile_fetch<D>(rg, gb + at, tid, rows, p.d);
+    if (DK) trans_fetch<D>(rqt, qb + at, tid, rows, p.d);
+    if (DV) trans_fetch<D>(rgt, gb + at, tid, rows, p.d);
+    if (tid < 2 * BT) {
+      const float* src = tid < BT ? lb : db;  // every lane loads; the factor is applied when stored
+      st = src[min(load.first_row() + (tid & (BT - 1)), p.sq - 1)];
     }
+    st_rows = rows;
+    load.next();
   };
   auto store = [&](int buf) {
-    unsigned char* base = smem + buf * BUF;
-    tile_store_rows<D>(rq, base);
-    if (DK) tile_store_rows<D>(rg, base + G::ROWMAJ);
-    if (DK) trans_store<D>(rqt, base + 2 * G::ROWMAJ);
-    if (DV) trans_store<D>(rgt, base + 2 * G::ROWMAJ + G::TRANS);
-    if (threadIdx.x < 2 * BT)
-      reinterpret_cast<float*>(base + 2 * G::ROWMAJ + 2 * G::TRANS)[threadIdx.x] = threadIdx.x < BT ? st * LOG2E : st;
+    unsigned char* base = lds + buf * BUF;
+    tile_store_rows<D>(rq, base, tid);
+    if (DK) tile_store_rows<D>(rg, base + G::ROWMAJ, tid);
+    if (DK) trans_store<D>(rqt, base + 2 * G::ROWMAJ, tid);
+    if (DV) trans_store<D>(rgt, base + 2 * G::ROWMAJ + G::TRANS, tid);
+    if (tid < 2 * BT) {
+      float v = tid < BT ? st * LOG2E : st;
+      if ((tid & (BT - 1)) >= st_rows) v = tid < BT ? INFINITY : 0.0f;  // a query past the end: probability 0
+      reinterpret_cast<float*>(base + 2 * G::ROWMAJ + 2 * G::TRANS)[tid] = v;
+    }
   };
-  fetch(0);
+  fetch();
   store(0);
-  // The fragments that came straight from memory are waited for here, once. Left to the first matrix
-  // instruction that reads them, the wait sits inside the loop, behind the tile loads every iteration has
-  // just issued, and counts those too: each iteration then waited for its own prefetch.
+  // waited for once, here (see the forward kernel)
 #pragma unroll
   for (int c = 0; c < G::C16; ++c) {
     asm volatile("" : "+v"(kf[c]));
@@ -506,12 +637,12 @@ __global__ __launch_bounds__(THREADS, (D <= 96 || MODE != 0) ? 2 : 1) void attn_
   }
   __syncthreads();
   for (int t = 0; t < ntiles; ++t) {
-    const unsigned char* qt = smem + (t & 1) * BUF;
+    const unsigned char* qt = lds + (t & 1) * BUF;
     const unsigned char* gt = qt + G::ROWMAJ;
     const unsigned char* qtt = qt + 2 * G::ROWMAJ;
     const unsigned char* gtt = qtt + G::TRANS;
     const float* stats = reinterpret_cast<const float*>(gtt + G::TRANS);
-    if (t + 1 < ntiles) fetch(t + 1);
+    if (t + 1 < ntiles) fetch();
     // S and dP: lane = key ln, register i = query 8*(i/4) + 4*kg + i%4 of the tile
     f32x16 s = zero16(), dp = zero16();
 #pragma unroll
@@ -550,18 +681,42 @@ __global__ __launch_bounds__(THREADS, (D <= 96 || MODE != 0) ? 2 : 1) void attn_
     if (t + 1 < ntiles) store((t + 1) & 1);
     __syncthreads();
   }
-  uint16_t* krow = p.dk + koff;
-  uint16_t* vrow = p.dv + koff;
+  if constexpr (KS > 1) {
+    static_assert(KS == 2 && MODE == 0 && WAVES * 32 * G::NB * 64 * 4 <= KS * 2 * BUF, "the hand-over reuses the stages");
+    float* xo = reinterpret_cast<float*>(smem) + wave * 32 * G::NB * 64 + lane;
+    if (ks == 1) {
+#pragma unroll
+      for (int nb = 0; nb < G::NB; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          xo[(nb * 16 + i) * 64] = dk[nb][i];
+          xo[((G::NB + nb) * 16 + i) * 64] = dv[nb][i];
+        }
+    }
+    __syncthreads();
+    if (ks == 1) return;
+#pragma unroll
+    for (int nb = 0; nb < G::NB; ++nb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        dk[nb][i] += xo[(nb * 16 + i) * 64];
+        dv[nb][i] += xo[((G::NB + nb) * 16 + i) * 64];
+      }
+  }
+  if (!live) return;
+  uint16_t* krow = reinterpret_cast<uint16_t*>(const_cast<char*>(chunk_entry(2, wg.chunk))) + koff;
+  uint16_t* vrow = reinterpret_cast<uint16_t*>(const_cast<char*>(chunk_entry(3, wg.chunk))) + koff;
 #pragma unroll
   for (int nb = 0; nb < G::NB; ++nb)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+      const int col = nb * 32 + 8 * j + 4 * kg;
+      if (col >= p.d) continue;
       if (DK)
-        *reinterpret_cast<u32x2*>(krow + nb * 32 + 8 * j + 4 * kg) =
-            pack4<F16>(dk[nb][4 * j] * p.scale, dk[nb][4 * j + 1] * p.scale, dk[nb][4 * j + 2] * p.scale,
-                       dk[nb][4 * j + 3] * p.scale);
+        *reinterpret_cast<u32x2*>(krow + col) = pack4<F16>(dk[nb][4 * j] * p.scale, dk[nb][4 * j + 1] * p.scale,
+                                                           dk[nb][4 * j + 2] * p.scale, dk[nb][4 * j + 3] * p.scale);
       if (DV)
-        *reinterpret_cast<u32x2*>(vrow + nb * 32 + 8 * j + 4 * kg) =
+        *reinterpret_cast<u32x2*>(vrow + col) =
             pack4<F16>(dv[nb][4 * j], dv[nb][4 * j + 1], dv[nb][4 * j + 2], dv[nb][4 * j + 3]);
     }
 }
@@ -579,41 +734,73 @@ int cu_count() {
   return cus;
 }
 
-template <int D, bool F16>
-int launch_fwd(const Args& a, long long batch, hipStream_t s) {
-  attn_wide_fwd_kernel<D, F16><<<dim3((unsigned)(a.sq / BQ), (unsigned)batch, 1), THREADS, 0, s>>>(a);
-  JG_CHECK_LAUNCH("jg_attn_fwd(wide)");
+// Groups per workgroup. A launch that leaves CUs without a workgroup splits the streamed side over more wavefronts
+// of one: up to 4 groups where the registers of 16 wavefronts hold the state (forward, D <= 64), else 2.
+int split_of(long long workgroups, int most) {
+  int ks = 1;
+  while (ks < most && workgroups * ks < cu_count()) ks *= 2;
+  return ks;
+}
+
+// `args` in a launch of `kernel` that needs more LDS than the default limit
+template <typename K>
+int launch(K kernel, dim3 grid, int threads, int lds, const ChunkTable& tab, const Args& a, hipStream_t s, const char* who) {
+  if (lds > 64 * 1024 &&
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, lds);
+  kernel<<<grid, threads, lds, s>>>(tab, a);
+  JG_CHECK_LAUNCH(who);
   return JG_OK;
 }
 
 template <int D, bool F16>
-int launch_bwd(const Args& a, long long batch, hipStream_t s) {
+int launch_fwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
+  typedef Geo<D> G;
+  constexpr int LDS = 2 * (G::ROWMAJ + G::TRANS);
+  const dim3 grid((unsigned)jg::cdiv(a.sq, BQ), (unsigned)batch, 1);
+  const char* who = "jg_attn_fwd(wide)";
+  const int ks = split_of((long long)grid.x * batch, D <= 64 ? 4 : 2);
+  if constexpr (D <= 64)
+    if (ks == 4) return launch(&attn_wide_fwd_kernel<D, F16, 4>, grid, 4 * GROUP, 4 * LDS, tab, a, s, who);
+  if (ks == 2) return launch(&attn_wide_fwd_kernel<D, F16, 2>, grid, 2 * GROUP, 2 * LDS, tab, a, s, who);
+  return launch(&attn_wide_fwd_kernel<D, F16, 1>, grid, GROUP, LDS, tab, a, s, who);
+}
+
+template <int D, bool F16>
+int launch_bwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
   typedef Geo<D> G;
   constexpr int DQ_LDS = 2 * (2 * G::ROWMAJ + G::TRANS);
   constexpr int DKV_LDS = 2 * (2 * G::ROWMAJ + 2 * G::TRANS + 2 * BT * 4);
-  void (*dqk)(Args) = &attn_wide_dq_kernel<D, F16>;
-  hipError_t e1 = hipFuncSetAttribute(reinterpret_cast<const void*>(dqk), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      DQ_LDS);
-  if (e1 != hipSuccess) JG_FAIL(JG_ERR_LAUNCH, "jg_attn_bwd(wide): cannot reserve LDS");
-  dqk<<<dim3((unsigned)(a.sq / BQ), (unsigned)batch, 1), THREADS, DQ_LDS, s>>>(a);
-  JG_CHECK_LAUNCH("jg_attn_bwd(wide, dq)");
-  // head size 96: dK and dV in one pass; head size 128: one pass each when the launch has more
-  // workgroups than the chip has CUs (register budget, see the kernel)
-  void (*passes[2])(Args) = {&attn_wide_dkv_kernel<D, F16, 0>, nullptr};
-  if constexpr (D > 96) {
-    if ((long long)(a.sk / BQ) * batch > cu_count()) {
-      passes[0] = &attn_wide_dkv_kernel<D, F16, 1>;
-      passes[1] = &attn_wide_dkv_kernel<D, F16, 2>;
-    }
+  const dim3 dq_grid((unsigned)jg::cdiv(a.sq, BQ), (unsigned)batch, 1);
+  const dim3 dkv_grid((unsigned)jg::cdiv(a.sk, BQ), (unsigned)batch, (unsigned)a.nchunks);
+  const long long dkv_workgroups = (long long)dkv_grid.x * batch * a.nchunks;
+  const char* who = "jg_attn_bwd(wide, dq)";
+  int rc = split_of((long long)dq_grid.x * batch, 2) == 2
+               ? launch(&attn_wide_dq_kernel<D, F16, 2>, dq_grid, 2 * GROUP, 2 * DQ_LDS, tab, a, s, who)
+               : launch(&attn_wide_dq_kernel<D, F16, 1>, dq_grid, GROUP, DQ_LDS, tab, a, s, who);
+  if (rc != JG_OK) return rc;
+  who = "jg_attn_bwd(wide, dkv)";
+  // up to head size 96: dK and dV in one pass; above: one pass each when the launch has more workgroups than the
+  // chip has CUs (register budget, see the kernel)
+  if constexpr (D <= 96) {
+    if (split_of(dkv_workgroups, 2) == 2)
+      return launch(&attn_wide_dkv_kernel<D, F16, 0, 2>, dkv_grid, 2 * GROUP, 2 * DKV_LDS, tab, a, s, who);
+  } else if (dkv_workgroups > cu_count()) {
+    rc = launch(&attn_wide_dkv_kernel<D, F16, 1, 1>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
+    if (rc != JG_OK) return rc;
+    return launch(&attn_wide_dkv_kernel<D, F16, 2, 1>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
   }
-  for (int i = 0; i < 2 && passes[i] != nullptr; ++i) {
-    hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void*>(passes[i]),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, DKV_LDS);
-    if (e2 != hipSuccess) JG_FAIL(JG_ERR_LAUNCH, "jg_attn_bwd(wide): cannot reserve LDS");
-    passes[i]<<<dim3((unsigned)(a.sk / BQ), (unsigned)batch, 1), THREADS, DKV_LDS, s>>>(a);
-    JG_CHECK_LAUNCH("jg_attn_bwd(wide, dkv)");
-  }
-  return JG_OK;
+  return launch(&attn_wide_dkv_kernel<D, F16, 0, 1>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
+}
+
+// f(D constant, F16 constant) for the narrowest kernel that holds the head
+template <typename F>
+int by_width(int d, int dtype, F f) {
+  auto typed = [&](auto width) { return dtype == JG_F16 ? f(width, std::true_type{}) : f(width, std::false_type{}); };
+  if (d <= 32) return typed(std::integral_constant<int, 32>{});
+  if (d <= 64) return typed(std::integral_constant<int, 64>{});
+  if (d <= 96) return typed(std::integral_constant<int, 96>{});
+  return typed(std::integral_constant<int, 128>{});
 }
 
 }  // namespace
@@ -621,42 +808,37 @@ int launch_bwd(const Args& a, long long batch, hipStream_t s) {
 namespace jg {
 
 bool attn_wide_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias) {
-  return (dtype == JG_BF16 || dtype == JG_F16) && !has_bias && (d == 96 || d == 128) && sq > 0 && sk > 0 && sq % BQ == 0 &&
-         sk % BQ == 0 && batch > 0 && batch <= 65535;
+  return (dtype == JG_BF16 || dtype == JG_F16) && !has_bias && d > 0 && d <= 128 && d % 8 == 0 && sq > 0 && sk > 0 &&
+         batch > 0 && batch <= 65535;
 }
 
-int attn_wide_fwd(void* out, float* lse, const void* q, const void* k, const void* v, long long batch, int sq,
-                  int sk, int d, int dtype, float scale, float* out_acc, float* lse_acc, hipStream_t s) {
+int attn_wide_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v, int nchunks,
+                         long long batch, int sq, int sk, int d, int dtype, float scale, float* out_acc, float* lse_acc,
+                         hipStream_t s) {
   Args a{};
   a.q = static_cast<const uint16_t*>(q);
-  a.k = static_cast<const uint16_t*>(k);
-  a.v = static_cast<const uint16_t*>(v);
   a.o = static_cast<uint16_t*>(out);
   a.lse = lse;
   a.out_acc = out_acc;
   a.lse_acc = lse_acc;
-  a.sq = sq; a.sk = sk; a.scale = scale;
-  if (dtype == JG_F16) return d == 128 ? launch_fwd<128, true>(a, batch, s) : launch_fwd<96, true>(a, batch, s);
-  return d == 128 ? launch_fwd<128, false>(a, batch, s) : launch_fwd<96, false>(a, batch, s);
+  a.sq = sq; a.sk = sk; a.d = d; a.nchunks = nchunks; a.scale = scale;
+  const ChunkTable tab = chunk_table(k, v, nullptr, nullptr, nchunks);
+  return by_width(d, dtype, [&](auto width, auto f16) { return launch_fwd<width(), f16()>(tab, a, batch, s); });
 }
 
-int attn_wide_bwd(void* dq, void* dk, void* dv, const void* dout, const void* q, const void* k, const void* v,
-                  const void* out, const float* lse, long long batch, int sq, int sk, int d, int dtype,
-                  float scale, void* ws, hipStream_t s) {
+int attn_wide_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q, const void* const* k,
+                         const void* const* v, int nchunks, const void* out, const float* lse, long long batch, int sq,
+                         int sk, int d, int dtype, float scale, void* ws, hipStream_t s) {
   Args a{};
   a.q = static_cast<const uint16_t*>(q);
-  a.k = static_cast<const uint16_t*>(k);
-  a.v = static_cast<const uint16_t*>(v);
   a.out = static_cast<const uint16_t*>(out);
   a.dout = static_cast<const uint16_t*>(dout);
   a.lse_in = lse;
   a.delta = static_cast<float*>(ws);
   a.dq = static_cast<uint16_t*>(dq);
-  a.dk = static_cast<uint16_t*>(dk);
-  a.dv = static_cast<uint16_t*>(dv);
-  a.sq = sq; a.sk = sk; a.scale = scale;
-  if (dtype == JG_F16) return d == 128 ? launch_bwd<128, true>(a, batch, s) : launch_bwd<96, true>(a, batch, s);
-  return d == 128 ? launch_bwd<128, false>(a, batch, s) : launch_bwd<96, false>(a, batch, s);
+  a.sq = sq; a.sk = sk; a.d = d; a.nchunks = nchunks; a.scale = scale;
+  const ChunkTable tab = chunk_table(k, v, dk, dv, nchunks);
+  return by_width(d, dtype, [&](auto width, auto f16) { return launch_bwd<width(), f16()>(tab, a, batch, s); });
 }
 
 }  // namespace jg

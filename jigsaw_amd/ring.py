@@ -54,7 +54,7 @@ from typing import Any
 
 import torch
 
-from .attention import attend_step_, backward_chunks, core_backward
+from .attention import _resident_backward, attend_step_, core_backward
 
 HopFn = Callable[..., "tuple[torch.Tensor, Any]"]
 
@@ -204,7 +204,7 @@ class RingSeat:
             if len(saved) != P:
                 raise ValueError(f"expected the {P} chunks the forward saved, got {len(saved)}")
             # every chunk is resident: one pass over all of them where the kernels cover it
-            one_pass = backward_chunks(dout, q, out, lse, [c[0].to(core) for c in saved], [c[1].to(core) for c in saved], scale)
+            one_pass = _resident_backward(dout, q, out, lse, [c[0] for c in saved], [c[1] for c in saved], scale)
             if one_pass is not None:
                 dq_all, dks, dvs = one_pass
                 dk_own = dv_own = None

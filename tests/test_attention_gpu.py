@@ -479,3 +479,40 @@ def test_head_sizes_between_the_kernel_sizes_are_zero_padded(d, dev):
     got = ja.backward(dout.to(dev), q.to(dev), k.to(dev), v.to(dev), want_o.float().to(dev), want_l.float().to(dev), scale, 33, 47)
     for g, w in zip(got, want):
         assert g.shape == w.shape and rel_l2(g, w) < 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,h,sq,sk,d,P", [
+    (1, 2, 1, 1, 64, 1), (1, 1, 129, 31, 64, 3), (2, 3, 127, 33, 64, 2), (1, 4, 300, 257, 64, 5), (1, 2, 128, 4097, 64, 1),
+    (1, 2, 1, 1, 32, 2), (1, 3, 130, 65, 8, 3), (2, 2, 100, 97, 40, 2), (1, 2, 257, 129, 80, 3), (1, 1, 33, 31, 96, 16),
+    (1, 2, 200, 300, 128, 2), (1, 40, 300, 260, 128, 2), (3, 90, 130, 100, 96, 1), (3, 90, 130, 100, 32, 1), (1, 5, 640, 513, 128, 1),
+], ids=str)
+def test_ring_of_any_lengths_in_one_pass(b, h, sq, sk, d, P, dtype, dev):
+    """Lengths at and beside the tile edges (32 keys, 64 rows, 128 resident rows), head sizes between the kernels' widths,
+    few and many workgroups (which split a workgroup's tiles over 1, 2 or 4 groups of wavefronts): forward and backward
+    over resident chunks against the oracle, and the fused merge of the same step against core + merge."""
+    torch.manual_seed(sq + sk + d)
+    q = (torch.randn(b, h, sq, d, device=dev) / d**0.5).to(dtype)
+    ks = [torch.randn(b, h, sk, d, device=dev).to(dtype) for _ in range(P)]
+    vs = [torch.randn(b, h, sk, d, device=dev).to(dtype) for _ in range(P)]
+    dout = torch.randn(b, h, sq, d, device=dev).to(dtype)
+    scale = d**-0.5
+    dbl = lambda t: t.double().cpu()  # noqa: E731
+    assert ja._resident(q, ks, vs)
+    out, lse = ja.ring_forward(q, ks, vs, scale, rank=P // 2)
+    want_o, want_l = oa.ring_forward(dbl(q), [dbl(t) for t in ks], [dbl(t) for t in vs], scale)
+    assert rel_l2(out, want_o) < 1e-2 and rel_l2(lse, want_l) < 1e-3
+    dq, dks, dvs = ja.ring_backward(dout, q, out, lse, ks, vs, scale)
+    parts = [oa.core_backward(dbl(dout), dbl(q), dbl(k), dbl(v), dbl(out), dbl(lse), scale) for k, v in zip(ks, vs)]
+    want_dq = sum(p[0] for p in parts)
+    if sk * P > 1:  # one key: dq and dk are zero in exact arithmetic
+        assert rel_l2(dq, want_dq) < 2e-2
+        assert rel_l2(torch.stack(dks), torch.stack([p[1] for p in parts])) < 2e-2
+    assert rel_l2(torch.stack(dvs), torch.stack([p[2] for p in parts])) < 2e-2
+    acc1, l1 = torch.randn(b, h, sq, d, device=dev), torch.randn(b, h, sq, device=dev)
+    acc2, l2 = acc1.clone(), l1.clone()
+    assert ja._fused_ok(q, ks[0])
+    acc1, l1 = ja.attend_step_(q, ks[0], vs[0], scale, acc1, l1)
+    o_j, l_j = ja.core_forward(q, ks[0], vs[0], scale)
+    acc2, l2 = ja.fused_online_softmax_merge_(acc2, l2, o_j, l_j, "bhsd")
+    assert rel_l2(acc1, acc2) < 1e-5 and rel_l2(l1, l2) < 1e-5
