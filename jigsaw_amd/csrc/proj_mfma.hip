@@ -18,10 +18,12 @@
 //   proj_tn_kernel   part[split](n, c) = sum_{r in split} g(r, n) * x(r, c)   (weight gradient;
 //                    bias gradient sum_r g(r, n) on the way), then proj_reduce_kernel
 //
-// bf16 on v_mfma_f32_32x32x16_bf16 with fp32 accumulation. Workgroup tile 128 x 128, four
-// wavefronts of 64 x 64 (2 x 2 MFMA blocks); operands are staged through LDS in 16-byte
-// slots of 8 contraction elements, fetched to registers one stage ahead of the MFMAs.
+// bf16 on v_mfma_f32_32x32x16_bf16 with fp32 accumulation. Workgroup tiles of 256 x 256 (eight wavefronts
+// of 128 x 64), 128 x 128 and, NT, 64 x 64 (four wavefronts); the operands travel from memory straight
+// into LDS, 64 contraction elements a stage, one stage ahead of the MFMAs.
 // proj_generic_kernel covers the other dtypes and unaligned shapes with plain FMAs.
+#include <type_traits>
+
 #include "jg_common.h"
 
 namespace {
@@ -89,7 +91,7 @@ struct NtParams {
   Map am, om;
   long long rows;
   int N, K;
-  int tiles_n;
+  int tiles_n, tiles;
   // What happens to a result on its way out (the values are the bf16-rounded acc + bias, as a
   // separate elementwise pass over the stored tensor would see them; arithmetic in fp32):
   //   EPI_NONE  out = y
@@ -142,101 +144,117 @@ __device__ __forceinline__ u32x4 map8(u32x4 y, u32x4 r, F f) {
   return u32x4{oo[0], oo[1], oo[2], oo[3]};
 }
 
+// ------------------------------------------------- memory -> LDS, both GEMMs
+// One wavefront instruction lands 64 x 16 bytes contiguously in LDS, in lane order; the source is a wave-uniform
+// base plus a 32-bit byte offset per lane (the host checks the tensor sizes), the LDS address of the 1 KB block goes
+// into M0. Written in assembly: with the compiler's own form it waits for ALL outstanding transfers before every
+// LDS read. The kernels order reads and transfers themselves, by one wait and one barrier per stage.
+__device__ __forceinline__ void dma_1k(const void* base, uint32_t lane_off, uint32_t lds_dst) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(base), "s"(lds_dst));
+}
+__device__ __forceinline__ uint32_t lds_address(const unsigned char* p) {
+  typedef __attribute__((address_space(3))) unsigned char* lds_bytes;
+  return (uint32_t)(uintptr_t)((lds_bytes)p);
+}
+__device__ __forceinline__ void transfers_landed() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // vmcnt(0)
+
 // Shape of a workgroup: WM x WN wavefronts, each with IM x JN blocks of 32 tokens x 32 features.
 template <int IM, int JN, int WM, int WN>
 struct NtShape {
   static constexpr int TM = 32 * IM * WM, TNF = 32 * JN * WN;  // tokens, features of a tile
-  static constexpr int THREADS = 64 * WM * WN;
-  static constexpr int OP_A = 8 * TM, OP_W = 8 * TNF;          // 16-byte slots per stage: [chunk of 8 k][row ^ 2 chunk]
-  static constexpr int STAGE = OP_A + OP_W;
-  static constexpr int OUT_PITCH = TNF + 8;                    // elements per token row of the result tile in LDS
-  static constexpr int MAIN = 2 * STAGE * 16 > TM * OUT_PITCH * 2 ? 2 * STAGE * 16 : TM * OUT_PITCH * 2;
-  static constexpr int LDS = MAIN + TNF * 4;                   // then the bias of the tile as floats
-  static constexpr int PASS_A = TM * 8 / THREADS, PASS_W = TNF * 8 / THREADS;
-  static_assert(TM * 8 % THREADS == 0 && TNF * 8 % THREADS == 0, "whole load passes");
+  static constexpr int WAVES = WM * WN, THREADS = 64 * WAVES;
+  static constexpr int ROWB = BK * 2;                          // bytes of a row of a stage: 8 chunks of 8 k, chunk c at c ^ (row % 8)
+  static constexpr int OP_A = TM * ROWB, OP_W = TNF * ROWB, STAGE = OP_A + OP_W;
+  static constexpr int LDS = 2 * STAGE + 2 * TNF * 4;          // two stages, then the bias of two tiles as floats
+  static constexpr int DMA_A = TM / 8 / WAVES, DMA_W = TNF / 8 / WAVES;  // 1 KB transfers (8 rows) of a wavefront per stage
+  static constexpr int OUT_PITCH = 32 * JN * 2 + 16;           // bytes per token of a wavefront's block in LDS
+  static_assert(TM % (8 * WAVES) == 0 && TNF % (8 * WAVES) == 0, "whole transfers");
+  static_assert(32 * OUT_PITCH * WAVES <= STAGE, "the results pass through the stage just computed");
 };
 
+// Persistent workgroups walk the tiles of one XCD's contiguous range (consecutive tiles share a panel of `a`, which
+// meets in one L2). The transfers of a stage are issued a stage ahead, across tile borders too, so that the first
+// stage of a tile arrives under the last one of the tile before and under its epilogue: with K = 512 a tile is only
+// eight stages long. Bound by the matrix cores and, beside them, by the LDS reads (3/4 KB per matrix instruction in
+// the 256 x 256 tile). 32768 tokens: 512 -> 1536 features 57.6 us (894 TFLOP/s; staged through registers, a tile per
+// workgroup: 68.1), 1536 -> 512 53.2 us (59.5), 512 -> 512 23.8 us (26.2); 65536 tokens, 128 -> 384 19.1 us (23.2).
 template <int IM, int JN, int WM, int WN>
-__global__ __launch_bounds__(64 * WM * WN) void proj_nt_kernel(NtParams p) {
+__global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_nt_kernel(NtParams p) {
   typedef NtShape<IM, JN, WM, WN> SH;
-  constexpr int TM = SH::TM, TNF = SH::TNF, THREADS = SH::THREADS;
+  constexpr int TM = SH::TM, TNF = SH::TNF, ROWB = SH::ROWB;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  u32x4* lds = reinterpret_cast<u32x4*>(smem);
+  float* lds_bias = reinterpret_cast<float*>(smem + 2 * SH::STAGE);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kg = lane >> 5;
   const int wm = wave % WM, wn = wave / WM;
-  // Workgroups go to the 8 XCDs round-robin; give each XCD a contiguous range of tiles, so that the
-  // tiles that share a panel of `a` (consecutive ids) meet in one L2.
-  const unsigned per_xcd = gridDim.x / 8;
-  const unsigned tile_id = blockIdx.x < per_xcd * 8 ? (blockIdx.x % 8) * per_xcd + blockIdx.x / 8 : blockIdx.x;
-  const long long m0 = (long long)(tile_id / p.tiles_n) * TM;
-  const int n0 = (tile_id % p.tiles_n) * TNF;
-  if (tid < TNF)  // read after the barriers of the stage loop
-    reinterpret_cast<float*>(smem + SH::MAIN)[tid] =
-        (p.bias != nullptr && n0 + tid < p.N) ? jg::bf16_to_f32(p.bias[n0 + tid]) : 0.0f;
+  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
 
-  // loads of a stage: chunk column c, rows tid / 8 + (THREADS / 8) i of both operands
-  constexpr int RSTEP = THREADS / 8;
-  const int c = tid & 7, lrow = tid >> 3;
-  // byte offsets from the start of a / w: 32 bits (the host checks the tensor sizes), so that a
-  // load takes the uniform base from scalar registers and one vector register per address
-  uint32_t a_row[SH::PASS_A], w_row[SH::PASS_W];
+  // tiles of this workgroup (the grid is a multiple of 8)
+  const int per_xcd = (p.tiles + 7) >> 3, wg_per_xcd = gridDim.x >> 3;
+  const int t_begin = (blockIdx.x & 7) * per_xcd, slot = blockIdx.x >> 3;
+  const int t_len = min(per_xcd, p.tiles - t_begin);
+  if (slot >= t_len) return;
+  const int my_tiles = (t_len - slot + wg_per_xcd - 1) / wg_per_xcd;
+  auto tile_at = [&](int i) { return t_begin + slot + i * wg_per_xcd; };
+
+  // ---- load cursor. Lane L of a transfer sits at row L / 8, chunk position L % 8, and fetches chunk
+  // (L % 8) ^ (row % 8), the same one in every transfer.
+  const int chunk = (lane & 7) ^ (lane >> 3);
+  uint32_t a_row[SH::DMA_A], w_row[SH::DMA_W];
+  int ld_tile = -1, ld_ks = 0;
+  uint16_t bias_next = 0;  // raw: converted when it goes to LDS, a use here would wait for the load
+  const int nk = (p.K + BK - 1) / BK;
+  auto enter_tile = [&]() {
+    ++ld_tile;
+    ld_ks = 0;
+    const int t = tile_at(ld_tile);
+    const long long m0 = (long long)(t / p.tiles_n) * TM;
+    const int n0 = (t % p.tiles_n) * TNF;
 #pragma unroll
-  for (int i = 0; i < SH::PASS_A; ++i) {
-    long long r = m0 + lrow + RSTEP * i;
-    if (r > p.rows - 1) r = p.rows - 1;  // a row past the end repeats the last one and is dropped
-    a_row[i] = (uint32_t)(row_part(p.am, r) * 2);
-  }
+    for (int i = 0; i < SH::DMA_A; ++i) {
+      long long r = m0 + (i * SH::WAVES + wave) * 8 + (lane >> 3);
+      if (r > p.rows - 1) r = p.rows - 1;  // a row past the end repeats the last one and is dropped
+      a_row[i] = (uint32_t)(row_part(p.am, r) * 2);
+    }
 #pragma unroll
-  for (int i = 0; i < SH::PASS_W; ++i) {
-    int n = n0 + lrow + RSTEP * i;
-    if (n > p.N - 1) n = p.N - 1;
-    w_row[i] = (uint32_t)((long long)n * p.K * 2);
-  }
-  const char* a_bytes = reinterpret_cast<const char*>(p.a);
-  const char* w_bytes = reinterpret_cast<const char*>(p.w);
-  u32x4 ra[SH::PASS_A], rw[SH::PASS_W];
-  bool ld_ok = true;
-  auto load = [&](int ks) {
-    const int k = ks * BK + c * 8;
-    ld_ok = k < p.K;  // a chunk past the contraction length is read at k = 0 and zeroed on the way to LDS
-    const int kk = ld_ok ? k : 0;
+    for (int i = 0; i < SH::DMA_W; ++i) {
+      const int n = min(n0 + (i * SH::WAVES + wave) * 8 + (lane >> 3), p.N - 1);
+      w_row[i] = (uint32_t)((long long)n * p.K * 2);
+    }
+    if (p.bias != nullptr) bias_next = p.bias[min(n0 + tid, p.N - 1)];  // features past the end are dropped
+  };
+  const uint32_t lds_a = lds_address(smem) + wave_u * 1024, lds_w = lds_a + SH::OP_A;
+  auto issue = [&](int buf) {
+    const int k = ld_ks * BK + chunk * 8;
+    const int kk = k < p.K ? k : 0;  // a chunk past the contraction length is read at k = 0 and zeroed below
     const uint32_t fa = (uint32_t)(feat_part(p.am, kk) * 2), fw = (uint32_t)kk * 2;
 #pragma unroll
-    for (int i = 0; i < SH::PASS_A; ++i) ra[i] = *reinterpret_cast<const u32x4*>(a_bytes + (size_t)(a_row[i] + fa));
+    for (int i = 0; i < SH::DMA_A; ++i) dma_1k(p.a, a_row[i] + fa, lds_a + buf * SH::STAGE + i * SH::WAVES * 1024);
 #pragma unroll
-    for (int i = 0; i < SH::PASS_W; ++i) rw[i] = *reinterpret_cast<const u32x4*>(w_bytes + (size_t)(w_row[i] + fw));
+    for (int i = 0; i < SH::DMA_W; ++i) dma_1k(p.w, w_row[i] + fw, lds_w + buf * SH::STAGE + i * SH::WAVES * 1024);
   };
-  auto store = [&](int buf) {
-    u32x4* sa = lds + buf * SH::STAGE;
-    u32x4* sw = sa + SH::OP_A;
-    const u32x4 zero = {0u, 0u, 0u, 0u};
+  // the last stage of a contraction length that is no multiple of BK: a lane clears what its transfers put past it
+  auto clear_tail = [&](int buf, int ks) {
+    if (ks * BK + chunk * 8 >= p.K) {
+      u32x4* at = reinterpret_cast<u32x4*>(smem + buf * SH::STAGE + wave * 1024 + lane * 16);
 #pragma unroll
-    for (int i = 0; i < SH::PASS_A; ++i) sa[c * TM + ((lrow + RSTEP * i) ^ (2 * c))] = ld_ok ? ra[i] : zero;
-#pragma unroll
-    for (int i = 0; i < SH::PASS_W; ++i) sw[c * TNF + ((lrow + RSTEP * i) ^ (2 * c))] = ld_ok ? rw[i] : zero;
+      for (int i = 0; i < SH::DMA_A + SH::DMA_W; ++i) at[i * SH::WAVES * 64] = u32x4{0u, 0u, 0u, 0u};
+    }
   };
 
   f32x16 acc[IM][JN];
-#pragma unroll
-  for (int i = 0; i < IM; ++i)
-#pragma unroll
-    for (int j = 0; j < JN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
   // acc[i][j] = w fragment (rows: features) x a fragment (columns: tokens). The fragments of
   // the next 16-wide step are requested before the MFMAs of this one are issued.
   auto compute = [&](int buf) {
-    const u32x4* sa = lds + buf * SH::STAGE;
-    const u32x4* sw = sa + SH::OP_A;
+    const unsigned char* sa = smem + buf * SH::STAGE + (wm * 32 * IM + ln) * ROWB;
+    const unsigned char* sw = smem + buf * SH::STAGE + SH::OP_A + (wn * 32 * JN + ln) * ROWB;
     u32x4 fr[2][IM + JN];
     auto fetch = [&](int kk, u32x4 (&f)[IM + JN]) {
-      const int cc = kk * 2 + kg;
+      const int at = ((kk * 2 + kg) ^ (ln & 7)) << 4;
 #pragma unroll
-      for (int t = 0; t < IM; ++t) f[t] = sa[cc * TM + ((wm * 32 * IM + t * 32 + ln) ^ (2 * cc))];
+      for (int t = 0; t < IM; ++t) f[t] = *reinterpret_cast<const u32x4*>(sa + t * 32 * ROWB + at);
 #pragma unroll
-      for (int t = 0; t < JN; ++t) f[IM + t] = sw[cc * TNF + ((wn * 32 * JN + t * 32 + ln) ^ (2 * cc))];
+      for (int t = 0; t < JN; ++t) f[IM + t] = *reinterpret_cast<const u32x4*>(sw + t * 32 * ROWB + at);
     };
     fetch(0, fr[0]);
 #pragma unroll
@@ -252,64 +270,88 @@ __global__ __launch_bounds__(64 * WM * WN) void proj_nt_kernel(NtParams p) {
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-
-  const int nk = (p.K + BK - 1) / BK;
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int ks = 0; ks < nk; ++ks) {
-    if (ks + 1 < nk) load(ks + 1);
-    compute(ks & 1);
-    if (ks + 1 < nk) store((ks + 1) & 1);
-    __syncthreads();
-  }
-
   // Accumulator lane (ln, kg), register e of block (i, j): feature (wn*JN + j)*32 + 8*(e/4) +
-  // 4*kg + e%4, token (wm*IM + i)*32 + ln. The tile goes to LDS as bf16 [token][feature]
-  // (the stages are done with), and leaves it in 16-byte pieces of 8 features.
-  uint16_t* tile = reinterpret_cast<uint16_t*>(smem);
-  const float* lds_bias = reinterpret_cast<const float*>(smem + SH::MAIN);
-#pragma unroll
-  for (int i = 0; i < IM; ++i)
+  // 4*kg + e%4, token (wm*IM + i)*32 + ln. The sums start from the bias.
+  auto init_acc = [&](int parity) {
+    const float* b = lds_bias + parity * TNF + wn * JN * 32 + kg * 4;
 #pragma unroll
     for (int j = 0; j < JN; ++j)
 #pragma unroll
       for (int e4 = 0; e4 < 4; ++e4) {
-        const int f = (wn * JN + j) * 32 + e4 * 8 + kg * 4;
-        const int tok = (wm * IM + i) * 32 + ln;
-        const f32x4 bq = *reinterpret_cast<const f32x4*>(lds_bias + f);
-        const f32x2 lo = {acc[i][j][e4 * 4 + 0] + bq.x, acc[i][j][e4 * 4 + 1] + bq.y};
-        const f32x2 hi = {acc[i][j][e4 * 4 + 2] + bq.z, acc[i][j][e4 * 4 + 3] + bq.w};
-        u32x2 pk;
-        pk.x = __builtin_bit_cast(uint32_t, __builtin_convertvector(lo, bf16x2));
-        pk.y = __builtin_bit_cast(uint32_t, __builtin_convertvector(hi, bf16x2));
-        *reinterpret_cast<u32x2*>(tile + tok * SH::OUT_PITCH + f) = pk;
+        const f32x4 bq = *reinterpret_cast<const f32x4*>(b + j * 32 + e4 * 8);
+#pragma unroll
+        for (int i = 0; i < IM; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][j][e4 * 4 + e] = bq[e];
       }
-  __syncthreads();
-  {
-    constexpr int CPR = TNF / 8, RPP = THREADS / CPR;  // 16-byte pieces per token row, rows per pass
-    const int fc = tid % CPR, trow = tid / CPR;
-    const int n = n0 + fc * 8;
+  };
+  // A wavefront's 32 tokens x 32 JN features pass through its slice of the stage just computed as bf16
+  // [token][feature] and leave in 16-byte pieces of 8 features, whole rows of 64 JN bytes at a time.
+  auto epilogue = [&](int t, int buf) {
+    unsigned char* block = smem + buf * SH::STAGE + wave * 32 * SH::OUT_PITCH;
+    constexpr int CPR = JN * 4, RPI = 64 / CPR;  // pieces per token, tokens per store instruction
+    const int fc = lane % CPR, trow = lane / CPR;
+    const int n = (t % p.tiles_n) * TNF + wn * 32 * JN + fc * 8;
+    const long long r0 = (long long)(t / p.tiles_n) * TM + wm * 32 * IM + trow;
     const long long fo = feat_part(p.om, n < p.N ? n : 0);
     RowWalk rwk;
-    rwk.start(p.om, m0 + trow);
-#pragma unroll 4
-    for (int q = 0; q < TM / RPP; ++q) {
-      const long long r = m0 + trow + RPP * q;
-      if (r < p.rows && n < p.N) {
-        const long long at = rwk.part(p.om) + fo;
-        u32x4 y = *reinterpret_cast<const u32x4*>(tile + (trow + RPP * q) * SH::OUT_PITCH + fc * 8);
-        if (p.epi == EPI_GELU) {
-          *reinterpret_cast<u32x4*>(p.aux + at) = map8(y, y, [](float h, float) { return gelu_f(h); });
-        } else if (p.epi == EPI_DGELU) {
-          y = map8(y, *reinterpret_cast<const u32x4*>(p.aux + at), [](float g, float h) { return g * dgelu_f(h); });
-        } else if (p.epi == EPI_ADD) {
-          y = map8(y, *reinterpret_cast<const u32x4*>(p.aux + at), [](float a, float b) { return a + b; });
+    rwk.start(p.om, r0);
+#pragma unroll
+    for (int i = 0; i < IM; ++i) {
+#pragma unroll
+      for (int j = 0; j < JN; ++j)
+#pragma unroll
+        for (int e4 = 0; e4 < 4; ++e4) {
+          const f32x2 lo = {acc[i][j][e4 * 4 + 0], acc[i][j][e4 * 4 + 1]}, hi = {acc[i][j][e4 * 4 + 2], acc[i][j][e4 * 4 + 3]};
+          u32x2 pk;
+          pk.x = __builtin_bit_cast(uint32_t, __builtin_convertvector(lo, bf16x2));
+          pk.y = __builtin_bit_cast(uint32_t, __builtin_convertvector(hi, bf16x2));
+          *reinterpret_cast<u32x2*>(block + ln * SH::OUT_PITCH + (j * 32 + e4 * 8 + kg * 4) * 2) = pk;
         }
-        *reinterpret_cast<u32x4*>(p.out + at) = y;
+      u32x4 piece[32 / RPI];
+#pragma unroll
+      for (int q = 0; q < 32 / RPI; ++q)
+        piece[q] = *reinterpret_cast<const u32x4*>(block + (trow + RPI * q) * SH::OUT_PITCH + fc * 16);
+#pragma unroll
+      for (int q = 0; q < 32 / RPI; ++q) {
+        if (r0 + i * 32 + RPI * q < p.rows && n < p.N) {
+          const long long at = rwk.part(p.om) + fo;
+          u32x4 y = piece[q];
+          if (p.epi == EPI_GELU) {
+            *reinterpret_cast<u32x4*>(p.aux + at) = map8(y, y, [](float h, float) { return gelu_f(h); });
+          } else if (p.epi == EPI_DGELU) {
+            y = map8(y, *reinterpret_cast<const u32x4*>(p.aux + at), [](float g, float h) { return g * dgelu_f(h); });
+          } else if (p.epi == EPI_ADD) {
+            y = map8(y, *reinterpret_cast<const u32x4*>(p.aux + at), [](float a, float b) { return a + b; });
+          }
+          *reinterpret_cast<u32x4*>(p.out + at) = y;
+        }
+        rwk.advance(p.om, RPI);
       }
-      rwk.advance(p.om, RPP);
     }
+  };
+
+  const bool tail = p.K % BK != 0;
+  enter_tile();
+  issue(0);
+  int buf = 0;
+  for (int ti = 0; ti < my_tiles; ++ti) {
+    for (int ks = 0; ks < nk; ++ks) {
+      transfers_landed();
+      if (tail && ks == nk - 1) clear_tail(buf, ks);
+      if (ks == 0 && tid < TNF) lds_bias[(ti & 1) * TNF + tid] = jg::bf16_to_f32(bias_next);
+      __syncthreads();  // stage ks is in LDS, and every wavefront is done with the other buffer
+      if (ks == 0) init_acc(ti & 1);
+      if (++ld_ks < nk) issue(buf ^ 1);
+      else if (ld_tile + 1 < my_tiles) {
+        enter_tile();
+        issue(buf ^ 1);
+      }
+      compute(buf);
+      buf ^= 1;
+    }
+    __syncthreads();  // the other wavefronts are done with the stage the results pass through
+    epilogue(tile_at(ti), buf ^ 1);
   }
 }
 
@@ -318,12 +360,19 @@ int launch_nt(NtParams& p, hipStream_t s, const char* who) {
   typedef NtShape<IM, JN, WM, WN> SH;
   p.tiles_n = jg::cdiv(p.N, SH::TNF);
   const long long tiles = (long long)jg::cdiv(p.rows, SH::TM) * p.tiles_n;
-  JG_REQUIRE(tiles < (1ll << 31), "%s: too many tiles", who);
+  JG_REQUIRE(tiles < (1ll << 30), "%s: too many tiles", who);
+  p.tiles = (int)tiles;
   void (*kern)(NtParams) = &proj_nt_kernel<IM, JN, WM, WN>;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     SH::LDS);
-  if (e != hipSuccess) JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, SH::LDS);
-  kern<<<(unsigned)tiles, SH::THREADS, SH::LDS, s>>>(p);
+  static bool reserved = false;
+  if (!reserved) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS) != hipSuccess)
+      JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, SH::LDS);
+    reserved = true;
+  }
+  // as many workgroups as fit at once (a multiple of 8: one share per XCD)
+  const long long fit = 256 * (160 * 1024 / SH::LDS);
+  const unsigned grid = (unsigned)(((tiles < fit ? tiles : fit) + 7) / 8 * 8);
+  kern<<<grid, SH::THREADS, SH::LDS, s>>>(p);
   JG_CHECK_LAUNCH(who);
   return JG_OK;
 }
@@ -339,148 +388,166 @@ struct TnParams {
   Map gm, xm;
   long long rows;
   int N, C;
-  int tiles_c;        // column tiles; blockIdx.x = (tile_n * tiles_c + tile_c), blockIdx.y = split
+  int tiles_c, tiles;  // column tiles, all tiles; a workgroup is split * tiles + tile_n * tiles_c + tile_c
   int stages_per_split;
 };
 
-// WM x WN wavefronts, each with IM x JN blocks of 32 features of g x 32 features of x; the tile is
-// square (T x T) and the workgroup has 2 T threads: one 8 token x 8 feature block per thread and stage.
+// WM x WN wavefronts, each with IM x JN blocks of 32 features of g x 32 features of x; the tile is square (T x T).
 template <int IM, int JN, int WM, int WN>
 struct TnShape {
   static constexpr int T = 32 * IM * WM;
-  static_assert(T == 32 * JN * WN, "square tile");
-  static constexpr int THREADS = 64 * WM * WN;
-  static_assert(THREADS == 2 * T, "one block per thread");
-  static constexpr int PITCH = T + T / 8;  // slots per chunk of 8 tokens: feature f at f + f / 8
-  static constexpr int OP = 8 * PITCH;
-  static constexpr int STAGE = 2 * OP;
-  static constexpr int LDS = 2 * STAGE * 16;
+  static_assert(T == 32 * JN * WN && IM == WN, "square tile; block i of the bias gradient goes to wavefront column i");
+  static constexpr int WAVES = WM * WN, THREADS = 64 * WAVES;
+  static constexpr int ROWB = 2 * T;                  // bytes of a token's row in LDS
+  static constexpr int OP = BR * ROWB, STAGE = 2 * OP, LDS = 2 * STAGE;
+  static constexpr int CPR = T / 8, RPI = 64 / CPR;   // 16-byte chunks per row, rows per transfer
+  static constexpr int DMA = OP / 1024 / WAVES;       // transfers of a wavefront per operand and stage
+  static constexpr int JROWS = WAVES * RPI;           // rows between a wavefront's transfers
 };
 
-// acc + the eight bf16 values of v. Plain shifts and adds: v_dot2c_f32_bf16 against a pair of ones is a
-// quarter of the instructions and gave the right sums by itself, but wrong ones in this kernel (chains of
-// dependent dot instructions), so it is not used.
-__device__ __forceinline__ float add_bf16x8(float acc, const u32x4& v) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    acc += __builtin_bit_cast(float, v[j] << 16);
-    acc += __builtin_bit_cast(float, v[j] & 0xffff0000u);
+// Tokens r, r + step, ... of an operand as byte offsets; heads: (b * H * S + s) * D, row-major: r * ld.
+struct TokenWalk {
+  uint32_t off;      // bytes
+  int s, S;          // position in the batch entry and its length
+  uint32_t row, jump;  // bytes between tokens of an entry; extra bytes from the end of an entry to the next one
+  __device__ __forceinline__ void start(const Map& m, long long r) {
+    row = (uint32_t)(m.heads ? m.D : m.ld) * 2u;
+    S = m.heads ? m.S : 0x7fffffff;
+    jump = m.heads ? (uint32_t)(m.H - 1) * (uint32_t)m.S * row : 0u;
+    const long long b = m.heads ? r / m.S : 0;
+    s = (int)(r - b * S);
+    off = (uint32_t)(row_part(m, r) * 2);
   }
-  return acc;
-}
+  __device__ __forceinline__ void advance(int by) {
+    s += by;
+    off += (uint32_t)by * row;
+    while (s >= S) {  // at most once where an entry is longer than the step
+      s -= S;
+      off += jump;
+    }
+  }
+};
 
-template <int IM, int JN, int WM, int WN, int AHEAD>
-__global__ __launch_bounds__(64 * WM * WN) void proj_tn_kernel(TnParams p) {
+// Weight gradient. The tiles of g and x (64 tokens x T features) lie in LDS as they lie in memory, a token per row,
+// brought there by direct transfers a stage ahead; the fragments, whose contraction runs over the tokens, come from
+// transposing LDS reads (ds_read_b64_tr_b16, as in the attention backward). Chunk c of a row sits at c ^ 4 (row % 4): the
+// four rows a transposing read of 16 lanes touches then cover all banks. No registers are staged and no vector
+// instruction transposes: with its reduction 92 us for 32768 tokens, 1536 x 512 (101 us with both), 1132 us for
+// 8192 x 8192 x 8192 (1294). A batch entry may be of any length: the octet-wise staging took multiples of 8 tokens
+// only and left the rest to the FMA kernel (5 x 590 tokens, 896 features, qkv and output projection: 2247 -> 250 us). The bias gradient is one more matrix instruction with ones, in the first column of tiles.
+template <int IM, int JN, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_kernel(TnParams p) {
   typedef TnShape<IM, JN, WM, WN> SH;
-  constexpr int T = SH::T;
+  constexpr int T = SH::T, ROWB = SH::ROWB;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  u32x4* lds = reinterpret_cast<u32x4*>(smem);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kg = lane >> 5;
   const int wn = wave % WM, wc = wave / WM;
-  const int tile_c = blockIdx.x % p.tiles_c, tile_n = blockIdx.x / p.tiles_c;
+  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  // Workgroups go to the 8 XCDs round-robin. The few tiles of 128 x 128 of a split are gathered on one XCD, where they
+  // meet in its L2 (65536 tokens, 512 x 128: 26.6 us, 29.5 spread). The 256-wide ones, which stream twice as much
+  // per workgroup, are spread (32768 tokens, 1536 x 512: 92 us, 113 gathered).
+  int id = blockIdx.x;
+  if (T == 128) {
+    const int per_xcd = gridDim.x / 8;
+    if (id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
+  }
+  const int split = id / p.tiles, tile = id - split * p.tiles;
+  const int tile_c = tile % p.tiles_c, tile_n = tile / p.tiles_c;
   const int n0 = tile_n * T, c0 = tile_c * T;
-  const int split = blockIdx.y;
   const long long r_first = (long long)split * p.stages_per_split * BR;
   long long r_last = r_first + (long long)p.stages_per_split * BR;
   if (r_last > p.rows) r_last = p.rows;
   const int nst = r_last > r_first ? (int)((r_last - r_first + BR - 1) / BR) : 0;
 
-  // loads: the first half of the threads fetches g, the second x; a thread owns an 8 token x 8 feature block
-  // `half` is the same for a whole wavefront (T is a multiple of 64). The operand's map is copied
-  // field by field: a reference chosen per thread (`half ? p.xm : p.gm`) made the compiler keep a
-  // pointer to the argument and re-read the fields from memory in every stage, each read followed by a
-  // wait for ALL outstanding loads, the staged ones included, which undid the lookahead below.
-  const int half = __builtin_amdgcn_readfirstlane(tid / T), tt = tid % T;
-  const int jc = tt % (T / 8), ro = tt / (T / 8);
-  Map mp;
-  mp.heads = half ? p.xm.heads : p.gm.heads;
-  mp.ld = half ? p.xm.ld : p.gm.ld;
-  mp.B = half ? p.xm.B : p.gm.B;
-  mp.H = half ? p.xm.H : p.gm.H;
-  mp.S = half ? p.xm.S : p.gm.S;
-  mp.D = half ? p.xm.D : p.gm.D;
-  const uint16_t* src = half ? p.x : p.g;
-  const int f_count = half ? p.C : p.N;
-  int f = (half ? c0 : n0) + jc * 8;
-  if (f > f_count - 8) f = f_count - 8;  // a block past the last feature repeats the last one and is dropped
-  const long long fpart = feat_part(mp, f);
-  RowWalk walk;
-  walk.start(mp, r_first + ro * 8);
-  const bool want_bias = (p.bias_part != nullptr) && half == 0 && tile_c == 0;
-  float bsum[8];
+  // ---- transfers: number j of a wavefront carries rows j * JROWS + wave * RPI + lane / CPR
+  const int my_row = wave * SH::RPI + lane / SH::CPR;
+  const int chunk = (lane % SH::CPR) ^ ((my_row & 3) << 2);  // JROWS is a multiple of 4: the same for every j
+  // a chunk past the last feature repeats the last one and is dropped
+  const uint32_t gf = (uint32_t)(feat_part(p.gm, min(n0 + chunk * 8, p.N - 8)) * 2);
+  const uint32_t xf = (uint32_t)(feat_part(p.xm, min(c0 + chunk * 8, p.C - 8)) * 2);
+  TokenWalk gw, xw;
+  gw.start(p.gm, min(r_first + my_row, p.rows - 1));
+  xw.start(p.xm, min(r_first + my_row, p.rows - 1));
+  const uint32_t lds_g = lds_address(smem) + wave_u * 1024;
+  auto issue = [&](int st, int buf) {
+    const long long left = p.rows - (r_first + (long long)st * BR);
+    const uint32_t dst = lds_g + buf * SH::STAGE;
+    if (left >= BR) {  // wave-uniform
+      TokenWalk a = gw, b = xw;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) bsum[j] = 0.0f;
-
-  // AHEAD register sets: the loads of stage st + AHEAD are issued at the head of stage st (into the set
-  // stage st was stored from), so a load has AHEAD - 1 whole stages to arrive before its registers go to
-  // LDS. With one set a workgroup moved 32 KB per memory latency: a stage's matrix instructions take a
-  // quarter of one.
-  u32x4 vs[AHEAD][8];
-  long long rl[AHEAD];
-  const uint32_t tok_stride32 = (uint32_t)(mp.heads ? mp.D : mp.ld);  // between consecutive tokens of one batch entry
-  uint32_t tok_off[8];
+      for (int j = 0; j < SH::DMA; ++j) {
+        dma_1k(p.g, a.off + gf, dst + j * SH::WAVES * 1024);
+        dma_1k(p.x, b.off + xf, dst + SH::OP + j * SH::WAVES * 1024);
+        a.advance(SH::JROWS);
+        b.advance(SH::JROWS);
+      }
+      gw = a;
+      xw = b;
+    } else {  // the stage the tokens end in: a row past the end repeats the last token and is cleared below
 #pragma unroll
-  for (int i = 0; i < 8; ++i) tok_off[i] = (uint32_t)i * tok_stride32;
-  auto load = [&](int st, u32x4 (&v)[8], long long& r_loaded) {
-    // tokens r_first + st*BR + ro*8 + i, all of one batch entry (S % 8 == 0); `walk` stands at i = 0.
-    // A token past the end repeats the last one (or token 0) and is zeroed on the way to LDS.
-    r_loaded = r_first + (long long)st * BR + ro * 8;
-    const long long left = p.rows - r_loaded;
-    const int last = left >= 8 ? 7 : (left > 0 ? (int)left - 1 : 0);
-    const uint16_t* b0 = src + (left > 0 ? walk.part(mp) : 0) + fpart;
-    // 32-bit element offsets inside the block of eight tokens (the host checks that 7 strides fit): the eight
-    // products are made once; a block cut short by the end of the tensor repeats its last token
-    const uint32_t last_off = (uint32_t)last * tok_stride32;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = *reinterpret_cast<const u32x4*>(b0 + (i < last ? tok_off[i] : last_off));
-    walk.advance(mp, BR);
-  };
-  auto store = [&](int buf, u32x4 (&v)[8], long long r_loaded, bool counted) {  // counted: a stage of this split
-    const bool add_bias = want_bias && counted;
-    u32x4* dst = lds + buf * SH::STAGE + half * SH::OP + ro * SH::PITCH + jc * 9;
-    if (r_loaded + 8 > p.rows) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (r_loaded + i >= p.rows) v[i] = u32x4{0u, 0u, 0u, 0u};
-    }
-#pragma unroll
-    for (int px = 0; px < 8; ++px) {
-      const uint32_t sel = (px & 1) ? 0x07060302u : 0x05040100u;
-      u32x4 t;
-      t.x = __builtin_amdgcn_perm(v[1][px >> 1], v[0][px >> 1], sel);
-      t.y = __builtin_amdgcn_perm(v[3][px >> 1], v[2][px >> 1], sel);
-      t.z = __builtin_amdgcn_perm(v[5][px >> 1], v[4][px >> 1], sel);
-      t.w = __builtin_amdgcn_perm(v[7][px >> 1], v[6][px >> 1], sel);
-      dst[px] = t;
-      if (add_bias) bsum[px] = add_bf16x8(bsum[px], t);
+      for (int j = 0; j < SH::DMA; ++j) {
+        const long long r = min(r_first + (long long)st * BR + j * SH::JROWS + my_row, p.rows - 1);
+        dma_1k(p.g, (uint32_t)(row_part(p.gm, r) * 2) + gf, dst + j * SH::WAVES * 1024);
+        dma_1k(p.x, (uint32_t)(row_part(p.xm, r) * 2) + xf, dst + SH::OP + j * SH::WAVES * 1024);
+      }
     }
   };
+  static_assert(SH::DMA * SH::JROWS == BR, "the walkers stand at the next stage after their transfers");
+  auto clear_tail = [&](int st, int buf) {
+    const int left = (int)(p.rows - (r_first + (long long)st * BR));
+    if (left >= BR) return;
+    u32x4* at = reinterpret_cast<u32x4*>(smem + buf * SH::STAGE + wave * 1024 + lane * 16);
+#pragma unroll
+    for (int j = 0; j < SH::DMA; ++j)
+      if (j * SH::JROWS + my_row >= left) {
+        at[j * SH::WAVES * 64] = u32x4{0u, 0u, 0u, 0u};
+        at[SH::OP / 16 + j * SH::WAVES * 64] = u32x4{0u, 0u, 0u, 0u};
+      }
+  };
 
-  f32x16 acc[IM][JN];
+  // ---- fragments: 32 features (block fb) x 16 tokens. Lane p of a group of 16 points at row 4 kg + p / 4, features
+  // 16 (group % 2) + 4 (p % 4) of the block; a second read takes the rows 8 further on.
+  auto frag_off = [&](int fb) {
+    const int pp = lane & 15, g1 = (lane >> 4) & 1;
+    const int c = 4 * fb + 2 * g1 + ((pp & 3) >> 1);
+    return (4 * kg + (pp >> 2)) * ROWB + ((c ^ ((pp >> 2) << 2)) << 4) + 8 * (pp & 1);
+  };
+  int g_off[IM], x_off[JN];
+#pragma unroll
+  for (int i = 0; i < IM; ++i) g_off[i] = frag_off(wn * IM + i);
+#pragma unroll
+  for (int j = 0; j < JN; ++j) x_off[j] = SH::OP + frag_off(wc * JN + j);
+  const int b_off = frag_off(wn * IM + wc);  // the block whose bias gradient this wavefront sums
+  auto tr_frag = [&](const unsigned char* at) {
+    typedef short i16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) i16x4* tr_ptr;
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at)));
+    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at + 8 * ROWB)));
+    return __builtin_bit_cast(bf16x8, u32x4{lo.x, lo.y, hi.x, hi.y});
+  };
+
+  f32x16 acc[IM][JN], acc_b;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc_b[e] = 0.0f;
 #pragma unroll
   for (int i = 0; i < IM; ++i)
 #pragma unroll
-    for (int j = 0; j < JN; ++j)
+    for (int j = 0; j < JN; ++j) acc[i][j] = acc_b;
+  bf16x8 ones;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  for (int e = 0; e < 8; ++e) ones[e] = (__bf16)1.0f;
 
-  auto compute = [&](int buf) {
-    const u32x4* sg = lds + buf * SH::STAGE;
-    const u32x4* sx = sg + SH::OP;
-    u32x4 fr[2][IM + JN];
-    auto fetch = [&](int kk, u32x4 (&fq)[IM + JN]) {
-      const int cc = kk * 2 + kg;
+  auto compute = [&](int buf, auto with_bias) {
+    const unsigned char* st = smem + buf * SH::STAGE;
+    bf16x8 fr[2][IM + JN + 1];
+    auto fetch = [&](int kk, bf16x8 (&f)[IM + JN + 1]) {
+      const unsigned char* at = st + kk * 16 * ROWB;
 #pragma unroll
-      for (int t = 0; t < IM; ++t) {
-        const int fg = (wn * IM + t) * 32 + ln;
-        fq[t] = sg[cc * SH::PITCH + fg + (fg >> 3)];
-      }
+      for (int t = 0; t < IM; ++t) f[t] = tr_frag(at + g_off[t]);
 #pragma unroll
-      for (int t = 0; t < JN; ++t) {
-        const int fx = (wc * JN + t) * 32 + ln;
-        fq[IM + t] = sx[cc * SH::PITCH + fx + (fx >> 3)];
-      }
+      for (int t = 0; t < JN; ++t) f[IM + t] = tr_frag(at + x_off[t]);
+      if (with_bias) f[IM + JN] = tr_frag(at + b_off);
     };
     fetch(0, fr[0]);
 #pragma unroll
@@ -491,40 +558,25 @@ __global__ __launch_bounds__(64 * WM * WN) void proj_tn_kernel(TnParams p) {
       for (int i = 0; i < IM; ++i)
 #pragma unroll
         for (int j = 0; j < JN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fr[kk & 1][i]),
-                                                              __builtin_bit_cast(bf16x8, fr[kk & 1][IM + j]), acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[kk & 1][i], fr[kk & 1][IM + j], acc[i][j], 0, 0, 0);
+      if (with_bias) acc_b = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[kk & 1][IM + JN], ones, acc_b, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  // stage st lives in register set st % AHEAD; the loop is unrolled AHEAD times so that the sets are named at
-  // compile time. Nothing in the main loop is conditional: a load or an LDS store under a condition made the
-  // compiler merge the set's old and new values through copies, and a copy waits for the load. Loads past the
-  // split's last stage read tokens that exist (clamped in `load`) and are never multiplied.
-#pragma unroll
-  for (int a = 0; a < AHEAD; ++a) load(a, vs[a], rl[a]);
-  store(0, vs[0], rl[0], nst > 0);
-  __syncthreads();
-  const int nst_main = nst - nst % AHEAD;
-  int st = 0;
-  for (; st < nst_main; st += AHEAD) {
-#pragma unroll
-    for (int a = 0; a < AHEAD; ++a) {
-      load(st + a + AHEAD, vs[a], rl[a]);
-      compute((st + a) & 1);
-      store((st + a + 1) & 1, vs[(a + 1) % AHEAD], rl[(a + 1) % AHEAD], st + a + 1 < nst);
-      __syncthreads();
+  const bool want_bias = p.bias_part != nullptr && tile_c == 0;  // uniform over the workgroup
+  auto run = [&](auto with_bias) {
+    if (nst > 0) issue(0, 0);
+    for (int st = 0; st < nst; ++st) {
+      transfers_landed();
+      if (st == nst - 1) clear_tail(st, st & 1);
+      __syncthreads();  // stage st is in LDS, and every wavefront is done with the other buffer
+      if (st + 1 < nst) issue(st + 1, (st + 1) & 1);
+      compute(st & 1, with_bias);
     }
-  }
-  // the last nst % AHEAD stages: their tokens are in the sets already, the first of them in LDS
-#pragma unroll
-  for (int a = 0; a < AHEAD - 1; ++a) {
-    if (st + a < nst) {  // uniform
-      compute((st + a) & 1);
-      if (st + a + 1 < nst) store((st + a + 1) & 1, vs[a + 1], rl[a + 1], true);
-      __syncthreads();
-    }
-  }
+  };
+  if (want_bias) run(std::true_type{});
+  else run(std::false_type{});
 
   // register e of block (i, j): row n0 + (wn*IM + i)*32 + 8*(e/4) + 4*kg + e%4, column c0 + (wc*JN + j)*32 + ln
   float* part = p.part + (size_t)split * p.N * p.C;
@@ -541,20 +593,11 @@ __global__ __launch_bounds__(64 * WM * WN) void proj_tn_kernel(TnParams p) {
         }
       }
     }
-
-  if (p.bias_part != nullptr && tile_c == 0) {  // uniform over the workgroup
-    float* red = reinterpret_cast<float*>(smem);  // [8 token octets][T features]; the stages are done with
-    if (half == 0) {
+  if (want_bias && ln == 0) {  // every column of acc_b holds the same sums
 #pragma unroll
-      for (int px = 0; px < 8; ++px) red[ro * T + jc * 8 + px] = bsum[px];
-    }
-    __syncthreads();
-    if (tid < T) {
-      float sum = 0.0f;
-#pragma unroll
-      for (int o = 0; o < 8; ++o) sum += red[o * T + tid];
-      // a clamped block would count the last features twice: only features of this tile are written
-      if (n0 + tid < p.N && (n0 + (tid & ~7) <= p.N - 8)) p.bias_part[(size_t)split * p.N + n0 + tid] = sum;
+    for (int e = 0; e < 16; ++e) {
+      const int n = n0 + (wn * IM + wc) * 32 + (e >> 2) * 8 + kg * 4 + (e & 3);
+      if (n < p.N) p.bias_part[(size_t)split * p.N + n] = acc_b[e];
     }
   }
 }
@@ -750,9 +793,6 @@ bool map_vec_ok(const Map& m, long long features) {
   if (features % 8 != 0) return false;
   return m.heads ? (m.D % 8 == 0) : (m.ld % 8 == 0);
 }
-// eight consecutive tokens starting at a multiple of 8 belong to one batch entry
-bool map_octets_ok(const Map& m) { return !m.heads || m.S % 8 == 0; }
-
 // Token ranges (splits) the contraction is cut into so that `tiles` tiles fill the chip; a
 // split is worth its partial tile from about 8 stages on.
 int splits_for(long long rows, int tiles, int target, bool small_tiles = false) {
@@ -783,13 +823,15 @@ template <int IM, int JN, int WM, int WN>
 int launch_tn(TnParams& p, int splits, hipStream_t s, const char* who) {
   typedef TnShape<IM, JN, WM, WN> SH;
   p.tiles_c = jg::cdiv(p.C, SH::T);
-  const int tiles = jg::cdiv(p.N, SH::T) * p.tiles_c;
-  // the 128-wide tile has the registers for three sets of staged loads, the 256-wide one for one
-  void (*kern)(TnParams) = &proj_tn_kernel<IM, JN, WM, WN, (IM * JN <= 4 ? 3 : 1)>;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     SH::LDS);
-  if (e != hipSuccess) JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, SH::LDS);
-  kern<<<dim3((unsigned)tiles, (unsigned)splits), SH::THREADS, SH::LDS, s>>>(p);
+  p.tiles = jg::cdiv(p.N, SH::T) * p.tiles_c;
+  void (*kern)(TnParams) = &proj_tn_kernel<IM, JN, WM, WN>;
+  static bool reserved = false;
+  if (!reserved) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS) != hipSuccess)
+      JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, SH::LDS);
+    reserved = true;
+  }
+  kern<<<(unsigned)p.tiles * (unsigned)splits, SH::THREADS, SH::LDS, s>>>(p);
   JG_CHECK_LAUNCH(who);
   return JG_OK;
 }
@@ -853,6 +895,8 @@ static int proj_nt_common(const char* who, void* out, void* aux, int epi, const 
   // the 256-wide tile only where its last column of tiles is more than half full
   const int waste = jg::cdiv(n_out, 256) * 256 - n_out;
   if (big_tiles >= 256 && waste < 128) return launch_nt<4, 2, 2, 4>(p, s, who);
+  // 64 x 64 where 128 x 128 tiles would leave most of the chip idle (468 tokens, 704 -> 2112: 7.9 us, 13.1 before)
+  if ((long long)jg::cdiv(rows, 128) * jg::cdiv(n_out, 128) < 128) return launch_nt<1, 1, 2, 2>(p, s, who);
   return launch_nt<2, 2, 2, 2>(p, s, who);
 }
 
@@ -894,8 +938,8 @@ int jg_proj_tn(void* gw, void* gb, const void* g, const void* x, int dtype, int 
   rc = make_map(&xm, x_heads, c, rows, B, H, S, D, who, "input");
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool fast = dtype == JG_BF16 && map_vec_ok(gm, n) && map_vec_ok(xm, c) && map_octets_ok(gm) &&
-                    map_octets_ok(xm) && aligned16(g) && aligned16(x);
+  const bool fast = dtype == JG_BF16 && map_vec_ok(gm, n) && map_vec_ok(xm, c) && aligned16(g) && aligned16(x) &&
+                    (unsigned long long)rows * n < (1ull << 31) && (unsigned long long)rows * c < (1ull << 31);
   if (!fast) {
     GenParams gp;
     gp.p = g; gp.q = x; gp.bias = nullptr; gp.out = gw;

@@ -253,3 +253,28 @@ def test_fused_projection_entry_refuses_what_it_has_no_kernel_for(dev):
     y = jp.gelu_mlp(xf, w.float(), None, w2, None)
     ref = torch.nn.functional.linear(torch.nn.functional.gelu(torch.nn.functional.linear(xf, w.float())), w2)
     assert rel_l2(y, ref) < 1e-5
+
+
+@pytest.mark.parametrize("b,s,c,n_out,heads", [
+    (1, 1, 8, 24, 1), (3, 5, 64, 192, 2), (2, 63, 72, 200, 1), (5, 117, 136, 264, 3), (1, 65, 64, 64, 2), (7, 129, 256, 512, 4),
+    (2, 4100, 512, 1536, 8), (9, 1001, 264, 768, 4),
+], ids=str)
+def test_gemm_tiles_with_remainders(b, s, c, n_out, heads, dev):
+    """Token counts beside the 64-token stages, batch entries that end inside a stage (and are shorter than one),
+    contraction lengths beside the 64-wide stages, features beside the 64 / 128 / 256-wide tiles: ``linear`` and
+    the head-layout projection, forward and all gradients, against fp32 matrix products."""
+    torch.manual_seed(s)
+    d = 8 * max(1, n_out // (24 * heads))
+    x = torch.randn(b, s, c, device=dev).bfloat16()
+    for fn, n in ((lambda t, w, bias: jp.linear(t, w, bias), n_out), (lambda t, w, bias: jp.qkv_projection(t, w, bias, heads), 3 * heads * d)):
+        w, bias = (torch.randn(n, c, device=dev) / c**0.5).bfloat16(), torch.randn(n, device=dev).bfloat16()
+        leaves = [t.detach().clone().requires_grad_() for t in (x, w, bias)]
+        y = fn(*leaves)
+        g = torch.randn_like(y)
+        got = torch.autograd.grad(y, leaves, g)
+        tokens = lambda t: t.float() if t.dim() == 3 else t.float().permute(1, 3, 0, 2, 4).reshape(b, s, n)  # noqa: E731
+        g2, x2 = tokens(g).reshape(-1, n), x.float().reshape(-1, c)
+        assert rel_l2(tokens(y).reshape(-1, n), x2 @ w.float().t() + bias.float()) < 1e-2
+        assert rel_l2(got[0].reshape(-1, c), g2 @ w.float()) < 1e-2
+        assert rel_l2(got[1], g2.t() @ x2) < 1e-2
+        assert rel_l2(got[2], g2.sum(0)) < 1e-2
