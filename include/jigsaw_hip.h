@@ -374,6 +374,17 @@ int jg_proj_nt(void* out, const void* a, const void* w, const void* bias, int dt
 int jg_proj_nt_fused(void* out, void* aux, int epilogue, const void* a, const void* w, const void* bias, int dtype,
                      int64_t rows, int n_out, int k_in, void* stream);
 
+/* The same with the input in the (t, B, H, S, D) layout of attention heads (a_heads = 1): the output projection of
+ * an attention branch with the residual sum around it. */
+int jg_proj_nt_fused_heads(void* out, void* aux, int epilogue, const void* a, const void* w, const void* bias, int dtype,
+                           int64_t rows, int n_out, int k_in, int a_heads, int B, int H, int S, int D, void* stream);
+
+/* dst[i] (rows, cols) = src[i] rounded to bf16 and, where dst_t[i] is not NULL, dst_t[i] (cols, rows) = its
+ * transpose, for n <= 16 contiguous fp32 matrices (a vector: rows = 1) in one launch: the parameters of a block
+ * under autocast. src, dst, dst_t, rows, cols are HOST arrays, read before the call returns. */
+int jg_cast_params(void* const* dst, void* const* dst_t, const void* const* src, const int32_t* rows, const int32_t* cols,
+                   int n, void* stream);
+
 /* gw[n][c] = sum_r g(r, n) * x(r, c)  (n, c) row-major, and gb[n] = sum_r g(r, n)
  * (gb may be NULL): weight and bias gradient of a projection (torch's
  * Linear backward; g = grad of the projection's output, x = its input).
@@ -588,6 +599,17 @@ int jg_attn_swin_bwd(void* dq, void* dk, void* dv, float* dtable, const void* do
                      const void* v, const void* out, const float* lse, const float* table, const uint8_t* side,
                      int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t d, float scale, int dtype,
                      void* workspace, size_t workspace_bytes, void* stream);
+
+/* The same on shifted windows of a grid that wraps inside this rank (examples/swin.py:206-208 with the roll of
+ * a group of one): the windows lie on the grid rolled by (-shift_y, -shift_x), 0 <= shift < gh, gw; q, k, v,
+ * out and the gradients stay in the order of the grid that is not rolled. */
+int jg_attn_swin_shifted_fwd(void* out, float* lse, const void* q, const void* k, const void* v, const float* table,
+                             const uint8_t* side, int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t shift_y,
+                             int64_t shift_x, int64_t d, float scale, int dtype, void* stream);
+int jg_attn_swin_shifted_bwd(void* dq, void* dk, void* dv, float* dtable, const void* dout, const void* q, const void* k,
+                             const void* v, const void* out, const float* lse, const float* table, const uint8_t* side,
+                             int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t shift_y, int64_t shift_x,
+                             int64_t d, float scale, int dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -177,6 +177,15 @@ SIGNATURES: dict[str, tuple] = {
         c_int,
         [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int, c_int, c_void_p],
     ),
+    "jg_proj_nt_fused_heads": (
+        c_int,
+        [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int, c_int, c_int, c_int, c_int,
+         c_int, c_int, c_void_p],
+    ),
+    "jg_cast_params": (
+        c_int,
+        [POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p), POINTER(c_int32), POINTER(c_int32), c_int, c_void_p],
+    ),
     "jg_proj_nt": (
         c_int,
         [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
@@ -242,6 +251,17 @@ SIGNATURES: dict[str, tuple] = {
         c_int,
         [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64,
          c_int64, c_float, c_int, c_void_p],
+    ),
+    "jg_attn_swin_shifted_fwd": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64,
+         c_int64, c_int64, c_int64, c_float, c_int, c_void_p],
+    ),
+    "jg_attn_swin_shifted_bwd": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+         c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_float, c_int, c_void_p, c_size_t,
+         c_void_p],
     ),
     "jg_attn_swin_bwd_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64, c_int64]),
     "jg_attn_swin_bwd": (

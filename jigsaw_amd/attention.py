@@ -425,27 +425,29 @@ class _SwinGridAttention(torch.autograd.Function):
     """Attention inside the 8 x 8 windows of a token grid. ``qkv`` is (3, B, heads, gh * gw, 32), the
     tokens in grid order, as the qkv projection writes it; relative-position bias from ``table``
     (225, heads) and the shift mask from the per-token codes ``side`` (windows, 64) are formed inside
-    the kernel (examples/swin.py:99-170). Differentiable in qkv and table; the gradient comes back
-    as one (3, ...) tensor, so that nothing is stacked or split on the way to the projection."""
+    the kernel (examples/swin.py:99-170). ``shift``: the windows lie on the grid rolled by minus this
+    along both axes (the grid wraps inside this rank). Differentiable in qkv and table; the gradient comes
+    back as one (3, ...) tensor, so that nothing is stacked or split on the way to the projection."""
 
     @staticmethod
-    def forward(ctx, qkv, table, side, grid):  # noqa: D102
+    def forward(ctx, qkv, table, side, grid, shift=0):  # noqa: D102
         lib = _lib.load()
         qkv = qkv.contiguous()
         table = table.detach().float().contiguous()
         _, images, heads, tokens, d = qkv.shape
         gh, gw = grid
         scale = d ** -0.5
-        out = torch.empty_like(qkv[0])
+        out = torch.empty(qkv.shape[1:], dtype=qkv.dtype, device=qkv.device)
         lse = torch.empty(images * heads * tokens, dtype=torch.float32, device=qkv.device)
-        rc = lib.jg_attn_swin_fwd(
-            _lib.ptr(out), _lib.ptr(lse), _lib.ptr(qkv[0]), _lib.ptr(qkv[1]), _lib.ptr(qkv[2]), _lib.ptr(table),
-            _lib.ptr(side), images, heads, gh, gw, d, float(scale), _lib.dtype_code(qkv.dtype),
+        q, part = qkv.data_ptr(), out.numel() * qkv.element_size()
+        rc = lib.jg_attn_swin_shifted_fwd(
+            _lib.ptr(out), _lib.ptr(lse), q, q + part, q + 2 * part, _lib.ptr(table),
+            _lib.ptr(side), images, heads, gh, gw, shift % gh, shift % gw, d, float(scale), _lib.dtype_code(qkv.dtype),
             _lib.stream_ptr(qkv.device),
         )
-        _lib.check(rc, "jg_attn_swin_fwd")
+        _lib.check(rc, "jg_attn_swin_shifted_fwd")
         ctx.save_for_backward(qkv, table, side, out, lse)
-        ctx.grid, ctx.scale = (gh, gw), scale
+        ctx.grid, ctx.scale, ctx.shift = (gh, gw), scale, shift
         return out
 
     @staticmethod
@@ -462,25 +464,27 @@ class _SwinGridAttention(torch.autograd.Function):
             dtable = torch.empty_like(table)
             ws_bytes = lib.jg_attn_swin_bwd_workspace_bytes(images, heads, gh, gw)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=qkv.device)
-        rc = lib.jg_attn_swin_bwd(
-            _lib.ptr(dqkv[0]), _lib.ptr(dqkv[1]), _lib.ptr(dqkv[2]), _lib.ptr(dtable), _lib.ptr(grad_out),
-            _lib.ptr(qkv[0]), _lib.ptr(qkv[1]), _lib.ptr(qkv[2]), _lib.ptr(out), _lib.ptr(lse), _lib.ptr(table),
-            _lib.ptr(side), images, heads, gh, gw, d, float(ctx.scale), _lib.dtype_code(qkv.dtype), _lib.ptr(ws),
-            ws_bytes, _lib.stream_ptr(qkv.device),
+        q, dq, part = qkv.data_ptr(), dqkv.data_ptr(), out.numel() * qkv.element_size()
+        rc = lib.jg_attn_swin_shifted_bwd(
+            dq, dq + part, dq + 2 * part, _lib.ptr(dtable), _lib.ptr(grad_out),
+            q, q + part, q + 2 * part, _lib.ptr(out), _lib.ptr(lse), _lib.ptr(table),
+            _lib.ptr(side), images, heads, gh, gw, ctx.shift % gh, ctx.shift % gw, d, float(ctx.scale),
+            _lib.dtype_code(qkv.dtype), _lib.ptr(ws), ws_bytes, _lib.stream_ptr(qkv.device),
         )
-        _lib.check(rc, "jg_attn_swin_bwd")
-        return dqkv, dtable, None, None
+        _lib.check(rc, "jg_attn_swin_shifted_bwd")
+        return dqkv, dtable, None, None, None
 
 
-def swin_grid_attention_packed(qkv, table, side, grid):
-    """:func:`swin_grid_attention` on the (3, B, heads, tokens, 32) tensor of the qkv projection."""
+def swin_grid_attention_packed(qkv, table, side, grid, shift=0):
+    """:func:`swin_grid_attention` on the (3, B, heads, tokens, 32) tensor of the qkv projection; ``shift``: on
+    the windows of the grid rolled by ``-shift`` along both axes, for a grid that is not split over ranks."""
     if qkv.dim() != 5 or qkv.shape[0] != 3 or not swin_grid_supported(qkv[0], grid, SWIN_WINDOW):
         raise NotImplementedError("swin_grid_attention: (3, B, heads, tokens, 32) bf16 and 8 x 8 windows only")
     if side is not None and (side.dtype != torch.uint8 or side.numel() != qkv.shape[-2]):
         raise ValueError("side must be a uint8 code per token, (windows, 64)")
     if table.shape != (225, qkv.shape[2]):
         raise ValueError(f"table must be (225, heads = {qkv.shape[2]}), got {tuple(table.shape)}")
-    return _SwinGridAttention.apply(qkv, table, side, grid)
+    return _SwinGridAttention.apply(qkv, table, side, grid, int(shift))
 
 
 def swin_grid_attention(q, k, v, table, side, grid):

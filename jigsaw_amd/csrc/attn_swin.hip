@@ -6,7 +6,10 @@
 //              in row-major grid order, which is what the qkv projection writes and the output
 //              projection reads. A wavefront takes one (image, window, head) entry and addresses
 //              the 64 token rows of its window in that grid (8 runs of 8 consecutive rows), so the
-//              window partition and its inverse are never materialised.
+//              window partition and its inverse are never materialised. Shifted windows: window position (y, x)
+//              holds grid token ((y + shift_y) % gh, (x + shift_x) % gw), so that a grid whose borders
+//              wrap inside this rank needs no roll before and after (four 16.8 MB passes a step of
+//              configuration 5, 33 us).
 //   Bias       table is (225, heads) fp32, row (qy - ky + 7) * 15 + (qx - kx + 7) for query (qy, qx)
 //              and key (ky, kx) of a window. The wavefront keeps its head's column in LDS (times
 //              log2 e); with the accumulator layout of S^T = K Q^T (a lane is one query, its
@@ -37,7 +40,8 @@ struct SwinArgs {
   const float* table;                      // (225, heads)
   const uint8_t* side;                     // (windows, 64) or NULL
   float* bins;                             // (entries, 2, 225) or NULL: table-gradient parts
-  int heads, gw, nwx, nwin;
+  int heads, gh, gw, nwx, nwin;
+  int shift_y, shift_x;                    // the windows lie on the grid rolled by minus this: 0 <= shift < gh, gw
   long long entries, tokens;
   float scale;
 };
@@ -57,7 +61,12 @@ __device__ inline Entry locate(const SwinArgs& p, long long e, int ln) {
   const int wy = r.win / p.nwx, wx = r.win - wy * p.nwx;
   r.base = (img * p.heads + r.head) * p.tokens * D;
 #pragma unroll
-  for (int b = 0; b < 2; ++b) r.rowoff[b] = ((wy * WIN + 4 * b + (ln >> 3)) * p.gw + wx * WIN + (ln & 7)) * D;
+  for (int b = 0; b < 2; ++b) {
+    int y = wy * WIN + 4 * b + (ln >> 3) + p.shift_y, x = wx * WIN + (ln & 7) + p.shift_x;
+    y -= y >= p.gh ? p.gh : 0;
+    x -= x >= p.gw ? p.gw : 0;
+    r.rowoff[b] = (y * p.gw + x) * D;
+  }
   return r;
 }
 
@@ -385,7 +394,10 @@ __global__ __launch_bounds__(256) void swin_bins_stage2(const float* __restrict_
   dtable[(size_t)i * heads + head] = acc;
 }
 
-int check(const char* who, int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t d, int dtype, float scale) {
+int check(const char* who, int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t shift_y, int64_t shift_x, int64_t d,
+          int dtype, float scale) {
+  JG_REQUIRE(shift_y >= 0 && shift_x >= 0 && shift_y < gh && shift_x < gw, "%s: shift (%lld, %lld) outside the %lld x %lld grid",
+             who, (long long)shift_y, (long long)shift_x, (long long)gh, (long long)gw);
   JG_REQUIRE(dtype == JG_BF16, "%s: bf16 only", who);
   JG_REQUIRE(d == D, "%s: head size %lld, built for %d", who, (long long)d, D);
   JG_REQUIRE(images >= 0 && heads >= 1 && gh >= WIN && gw >= WIN && gh % WIN == 0 && gw % WIN == 0,
@@ -401,8 +413,12 @@ bool al16(std::initializer_list<const void*> ptrs) {
   return true;
 }
 
-SwinArgs common(int64_t images, int64_t heads, int64_t gh, int64_t gw, float scale, const float* table, const uint8_t* side) {
+SwinArgs common(int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t shift_y, int64_t shift_x, float scale,
+                const float* table, const uint8_t* side) {
   SwinArgs a = {};
+  a.gh = (int)gh;
+  a.shift_y = (int)shift_y;
+  a.shift_x = (int)shift_x;
   a.table = table;
   a.side = side;
   a.heads = (int)heads;
@@ -419,15 +435,16 @@ SwinArgs common(int64_t images, int64_t heads, int64_t gh, int64_t gw, float sca
 
 // Windowed attention of a Swin block on the token grid (examples/swin.py:129-170 with the index of
 // 99-104 and the mask of 107-126 formed in the kernel). lse: (images * windows * heads, 64) fp32.
-extern "C" int jg_attn_swin_fwd(void* out, float* lse, const void* q, const void* k, const void* v, const float* table,
-                                const uint8_t* side, int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t d,
-                                float scale, int dtype, void* stream) {
+extern "C" int jg_attn_swin_shifted_fwd(void* out, float* lse, const void* q, const void* k, const void* v,
+                                        const float* table, const uint8_t* side, int64_t images, int64_t heads, int64_t gh,
+                                        int64_t gw, int64_t shift_y, int64_t shift_x, int64_t d, float scale, int dtype,
+                                        void* stream) {
   const char* who = "jg_attn_swin_fwd";
-  int rc = check(who, images, heads, gh, gw, d, dtype, scale);
+  int rc = check(who, images, heads, gh, gw, shift_y, shift_x, d, dtype, scale);
   if (rc) return rc;
   JG_REQUIRE(out && lse && q && k && v && table, "%s: NULL pointer", who);
   JG_REQUIRE(al16({out, q, k, v}), "%s: tensors must be 16-byte aligned", who);
-  SwinArgs a = common(images, heads, gh, gw, scale, table, side);
+  SwinArgs a = common(images, heads, gh, gw, shift_y, shift_x, scale, table, side);
   if (a.entries == 0) return JG_OK;
   a.q = static_cast<const uint16_t*>(q);
   a.k = static_cast<const uint16_t*>(k);
@@ -448,16 +465,17 @@ extern "C" size_t jg_attn_swin_bwd_workspace_bytes(int64_t images, int64_t heads
   return (entries + (size_t)heads * CHUNKS) * BINS * sizeof(float);
 }
 
-extern "C" int jg_attn_swin_bwd(void* dq, void* dk, void* dv, float* dtable, const void* dout, const void* q, const void* k,
-                                const void* v, const void* out, const float* lse, const float* table, const uint8_t* side,
-                                int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t d, float scale, int dtype,
-                                void* workspace, size_t workspace_bytes, void* stream) {
+extern "C" int jg_attn_swin_shifted_bwd(void* dq, void* dk, void* dv, float* dtable, const void* dout, const void* q,
+                                        const void* k, const void* v, const void* out, const float* lse,
+                                        const float* table, const uint8_t* side, int64_t images, int64_t heads, int64_t gh,
+                                        int64_t gw, int64_t shift_y, int64_t shift_x, int64_t d, float scale, int dtype,
+                                        void* workspace, size_t workspace_bytes, void* stream) {
   const char* who = "jg_attn_swin_bwd";
-  int rc = check(who, images, heads, gh, gw, d, dtype, scale);
+  int rc = check(who, images, heads, gh, gw, shift_y, shift_x, d, dtype, scale);
   if (rc) return rc;
   JG_REQUIRE(dq && dk && dv && dout && q && k && v && out && lse && table, "%s: NULL pointer", who);
   JG_REQUIRE(al16({dq, dk, dv, dout, q, k, v, out}), "%s: tensors must be 16-byte aligned", who);
-  SwinArgs a = common(images, heads, gh, gw, scale, table, side);
+  SwinArgs a = common(images, heads, gh, gw, shift_y, shift_x, scale, table, side);
   if (a.entries == 0) return JG_OK;
   if (dtable != nullptr && (workspace == nullptr || workspace_bytes < jg_attn_swin_bwd_workspace_bytes(images, heads, gh, gw)))
     JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, workspace_bytes,
@@ -495,4 +513,18 @@ extern "C" int jg_attn_swin_bwd(void* dq, void* dk, void* dv, float* dtable, con
     JG_CHECK_LAUNCH(who);
   }
   return JG_OK;
+}
+
+extern "C" int jg_attn_swin_fwd(void* out, float* lse, const void* q, const void* k, const void* v, const float* table,
+                                const uint8_t* side, int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t d,
+                                float scale, int dtype, void* stream) {
+  return jg_attn_swin_shifted_fwd(out, lse, q, k, v, table, side, images, heads, gh, gw, 0, 0, d, scale, dtype, stream);
+}
+
+extern "C" int jg_attn_swin_bwd(void* dq, void* dk, void* dv, float* dtable, const void* dout, const void* q, const void* k,
+                                const void* v, const void* out, const float* lse, const float* table, const uint8_t* side,
+                                int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t d, float scale, int dtype,
+                                void* workspace, size_t workspace_bytes, void* stream) {
+  return jg_attn_swin_shifted_bwd(dq, dk, dv, dtable, dout, q, k, v, out, lse, table, side, images, heads, gh, gw, 0, 0, d,
+                                  scale, dtype, workspace, workspace_bytes, stream);
 }

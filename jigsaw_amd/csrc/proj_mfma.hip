@@ -772,6 +772,42 @@ __global__ __launch_bounds__(256) void proj_colsum_kernel(void* gb, const void* 
   }
 }
 
+// fp32 matrices to bf16 and to their transposes, a 64 x 64 tile per block, every matrix of the list in one launch
+// (a block's parameters are a few hundred KB: what a cast costs is its launch)
+constexpr int CAST_MOST = 16;
+struct CastArgs {
+  const float* src[CAST_MOST];
+  uint16_t* dst[CAST_MOST];
+  uint16_t* dst_t[CAST_MOST];
+  int rows[CAST_MOST], cols[CAST_MOST];
+  int end[CAST_MOST];  // blocks of this matrix and the ones before it
+};
+__global__ __launch_bounds__(256) void cast_params_kernel(CastArgs a) {
+  __shared__ uint16_t tile[64][66];
+  int m = 0;
+  while ((int)blockIdx.x >= a.end[m]) ++m;
+  const int t = blockIdx.x - (m == 0 ? 0 : a.end[m - 1]);
+  const int rows = a.rows[m], cols = a.cols[m], tiles_c = (cols + 63) / 64;
+  const int r0 = t / tiles_c * 64, c0 = t % tiles_c * 64;
+  const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+  const float* src = a.src[m];
+  uint16_t* dst = a.dst[m];
+  float v[16];  // all loads first: one memory latency a tile
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = src[(size_t)min(r0 + y + 4 * i, rows - 1) * cols + min(c0 + x, cols - 1)];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int r = y + 4 * i;
+    const uint16_t h = jg::f32_to_bf16(v[i]);
+    if (r0 + r < rows && c0 + x < cols) dst[(size_t)(r0 + r) * cols + c0 + x] = h;
+    tile[r][x] = h;
+  }
+  if (a.dst_t[m] == nullptr) return;
+  __syncthreads();
+  for (int i = y; i < 64; i += 4)
+    if (c0 + i < cols && r0 + x < rows) a.dst_t[m][(size_t)(c0 + i) * rows + r0 + x] = tile[x][i];
+}
+
 // --------------------------------------------------------------------- host
 int make_map(Map* m, int heads, long long features, long long rows, int B, int H, int S, int D, const char* who,
              const char* what) {
@@ -906,13 +942,42 @@ int jg_proj_nt(void* out, const void* a, const void* w, const void* bias, int dt
                         B, H, S, D, stream);
 }
 
-int jg_proj_nt_fused(void* out, void* aux, int epilogue, const void* a, const void* w, const void* bias, int dtype,
-                     int64_t rows, int n_out, int k_in, void* stream) {
+int jg_proj_nt_fused_heads(void* out, void* aux, int epilogue, const void* a, const void* w, const void* bias, int dtype,
+                           int64_t rows, int n_out, int k_in, int a_heads, int B, int H, int S, int D, void* stream) {
   const char* who = "jg_proj_nt_fused";
   JG_REQUIRE(epilogue == EPI_GELU || epilogue == EPI_DGELU || epilogue == EPI_ADD, "%s: unknown epilogue %d", who,
              epilogue);
   JG_REQUIRE(aux != nullptr && aligned16(aux), "%s: aux must be a 16-byte aligned tensor of the shape of out", who);
-  return proj_nt_common(who, out, aux, epilogue, a, w, bias, dtype, rows, n_out, k_in, 0, 0, 1, 1, 1, 1, stream);
+  return proj_nt_common(who, out, aux, epilogue, a, w, bias, dtype, rows, n_out, k_in, a_heads, 0, B, H, S, D, stream);
+}
+
+int jg_proj_nt_fused(void* out, void* aux, int epilogue, const void* a, const void* w, const void* bias, int dtype,
+                     int64_t rows, int n_out, int k_in, void* stream) {
+  return jg_proj_nt_fused_heads(out, aux, epilogue, a, w, bias, dtype, rows, n_out, k_in, 0, 1, 1, 1, 1, stream);
+}
+
+int jg_cast_params(void* const* dst, void* const* dst_t, const void* const* src, const int32_t* rows, const int32_t* cols,
+                   int n, void* stream) {
+  const char* who = "jg_cast_params";
+  JG_REQUIRE(n >= 0 && n <= CAST_MOST, "%s: at most %d tensors, got %d", who, CAST_MOST, n);
+  JG_REQUIRE(n == 0 || (dst && dst_t && src && rows && cols), "%s: null pointer", who);
+  CastArgs a = {};
+  long long blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    JG_REQUIRE(dst[i] && src[i] && rows[i] >= 0 && cols[i] >= 0, "%s: tensor %d", who, i);
+    a.src[i] = static_cast<const float*>(src[i]);
+    a.dst[i] = static_cast<uint16_t*>(dst[i]);
+    a.dst_t[i] = static_cast<uint16_t*>(dst_t[i]);
+    a.rows[i] = rows[i];
+    a.cols[i] = cols[i];
+    blocks += (long long)jg::cdiv(rows[i], 64) * jg::cdiv(cols[i], 64);
+    JG_REQUIRE(blocks < (1ll << 31), "%s: too large", who);
+    a.end[i] = (int)blocks;
+  }
+  if (blocks == 0) return JG_OK;
+  cast_params_kernel<<<(unsigned)blocks, 256, 0, static_cast<hipStream_t>(stream)>>>(a);
+  JG_CHECK_LAUNCH(who);
+  return JG_OK;
 }
 
 size_t jg_proj_tn_workspace(int64_t rows, int n, int c) {

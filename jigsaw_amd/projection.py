@@ -19,6 +19,7 @@ gradient: one GEMM contracted over the tokens). The weights are the rank's local
 from __future__ import annotations
 
 import contextlib
+import ctypes
 import math
 
 import torch
@@ -51,6 +52,11 @@ def remember_casts(on: bool = True) -> bool:
     global _remember_casts
     before, _remember_casts = _remember_casts, bool(on)
     return before
+
+
+def casts_remembered() -> bool:
+    """Whether :func:`remember_casts` is on."""
+    return _remember_casts
 
 
 def invalidate_casts(*targets) -> None:
@@ -111,9 +117,35 @@ def _cast_cached(t: torch.Tensor | None, dtype: torch.dtype, transposed: bool = 
     return got
 
 
+def cast_parameters(weights, biases) -> tuple:
+    """``(bf16 weights, their transposes, bf16 biases)`` of fp32 matrices and vectors, all in one launch
+    (``jg_cast_params``) into one buffer: a cast or a transpose of a parameter costs its launch."""
+    sizes = [t.numel() for t in (*weights, *weights, *biases)]
+    flat = torch.empty(sum((n + 7) // 8 * 8 for n in sizes), dtype=torch.bfloat16, device=weights[0].device)
+    views, at = [], 0
+    for t, n, transposed in zip((*weights, *weights, *biases), sizes, [False] * len(weights) + [True] * len(weights) + [False] * len(biases)):
+        shape = (t.shape[1], t.shape[0]) if transposed else tuple(t.shape)
+        views.append(flat.as_strided(shape, (shape[1], 1) if len(shape) == 2 else (1,), at))
+        at += (n + 7) // 8 * 8
+    k = len(weights)
+    w, wt, b = views[:k], views[k:2 * k], views[2 * k:]
+    n = k + len(biases)
+    src = (ctypes.c_void_p * n)(*[t.data_ptr() for t in (*weights, *biases)])
+    dst = (ctypes.c_void_p * n)(*[t.data_ptr() for t in (*w, *b)])
+    dst_t = (ctypes.c_void_p * n)(*[t.data_ptr() for t in wt])
+    rows = (ctypes.c_int32 * n)(*[t.shape[0] for t in weights], *[1] * len(biases))
+    cols = (ctypes.c_int32 * n)(*[t.shape[1] for t in weights], *[t.shape[0] for t in biases])
+    rc = _lib.load().jg_cast_params(dst, dst_t, src, rows, cols, n, _lib.stream_ptr(flat.device))
+    _lib.check(rc, "jg_cast_params")
+    return w, wt, b
+
+
 def _transposed(ctx, w: torch.Tensor) -> torch.Tensor:
-    """The transposed weight of the input-gradient GEMM: the remembered copy of the parameter when casts
-    are remembered and the parameter is still the one the forward saw, else a transpose of the saved cast."""
+    """The transposed weight of the input-gradient GEMM: what came with the cast (:func:`cast_parameters`), the
+    remembered copy of the parameter when casts are remembered and the parameter is still the one the forward
+    saw, else a transpose of the saved cast."""
+    if getattr(ctx, "weight_t", None) is not None:
+        return ctx.weight_t
     ref = getattr(ctx, "weight_ref", None)
     if _remember_casts and ref is not None and ref._version == ctx.weight_version:
         return _cast_cached(ref, w.dtype, transposed=True)
@@ -193,11 +225,12 @@ class _QkvProjection(torch.autograd.Function):
 
 
 class _HeadsProjection(torch.autograd.Function):
-    """``(*lead, h, s, d) -> (*lead, s, n_out)`` with ``weight (n_out, h d)``."""
+    """``(*lead, h, s, d) -> (*lead, s, n_out)`` with ``weight (n_out, h d)``; ``residual`` (contiguous, of the
+    result's shape and dtype, bf16) is added to the rounded result on the way out."""
 
     @staticmethod
-    def forward(ctx, out, weight, bias):  # noqa: D102
-        _lib.require_gpu(out, weight, bias)
+    def forward(ctx, out, weight, bias, residual=None):  # noqa: D102
+        _lib.require_gpu(out, weight, bias, residual)
         if out.dim() < 3:
             raise ValueError("out must be (..., heads, seq, head_dim)")
         n_out, k = weight.shape
@@ -210,7 +243,13 @@ class _HeadsProjection(torch.autograd.Function):
         w = _cast_cached(weight, out.dtype)
         bs = _cast_cached(bias, out.dtype)
         y = torch.empty((*lead, s, n_out), dtype=out.dtype, device=out.device)
-        if b * s:
+        ctx.has_residual = residual is not None
+        if b * s and residual is not None:
+            rc = _lib.load().jg_proj_nt_fused_heads(
+                _lib.ptr(y), _lib.ptr(residual), EPI_ADD, _lib.ptr(oc), _lib.ptr(w), _lib.ptr(bs), _lib.dtype_code(oc.dtype),
+                b * s, n_out, k, 1, b, h, s, d, _lib.stream_ptr(oc.device))
+            _lib.check(rc, "jg_proj_nt_fused_heads")
+        elif b * s:
             _nt(y, oc, w, bs, b * s, n_out, k, True, False, (b, h, s, d))
         ctx.save_for_backward(oc, w)
         ctx.weight_ref, ctx.weight_version = weight, weight._version
@@ -239,7 +278,7 @@ class _HeadsProjection(torch.autograd.Function):
                 gw, gb = _tn(g, oc, b * s, n_out, k, False, True, ctx.dims, need_b, _grad_dtype(g.dtype, ctx.dtypes))
         dt_w, dt_b = ctx.dtypes
         return (go, None if gw is None or not ctx.needs_input_grad[1] else gw.to(dt_w),
-                None if gb is None else gb.to(dt_b))
+                None if gb is None else gb.to(dt_b), grad if ctx.has_residual else None)
 
 
 class _Linear(torch.autograd.Function):
@@ -351,6 +390,8 @@ class _GeluMlp(torch.autograd.Function):
         dt_w1, dt_b1, dt_w2, dt_b2 = ctx.dtypes
 
         def transposed(i, wc):
+            if getattr(ctx, "weights_t", None) is not None:
+                return ctx.weights_t[i]
             ref, version = ctx.refs[i]
             return _cast_cached(ref, wc.dtype, transposed=True) if _remember_casts and ref._version == version else wc.t().contiguous()
 
@@ -386,7 +427,18 @@ def qkv_projection(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | N
 def heads_projection(out: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """``F.linear(rearrange(out, "... h s d -> ... s (h d)"), weight, bias)`` without the
     contiguous copy of the rearranged tensor (_attention.py:909-916)."""
-    return _HeadsProjection.apply(out, weight, bias)
+    return _HeadsProjection.apply(out, weight, bias, None)
 
 
-__all__ = ["gelu_mlp", "heads_projection", "invalidate_casts", "linear", "mlp_fusable", "qkv_projection", "remember_casts"]
+def heads_projection_add(out, weight, bias, residual) -> torch.Tensor:
+    """``residual + heads_projection(out, weight, bias)`` with the sum on the GEMM's way out where that exists
+    (bf16, feature counts that are multiples of 8), else in a step of its own."""
+    n_out, k = weight.shape
+    if (out.dtype == torch.bfloat16 and residual.dtype == torch.bfloat16 and residual.is_contiguous() and out.numel() > 0
+            and residual.data_ptr() % 16 == 0 and n_out % 8 == 0 and out.shape[-1] % 8 == 0
+            and tuple(residual.shape) == (*out.shape[:-3], out.shape[-2], n_out)):
+        return _HeadsProjection.apply(out, weight, bias, residual)
+    return residual + heads_projection(out, weight, bias).to(residual.dtype)
+
+
+__all__ = ["cast_parameters", "gelu_mlp", "heads_projection", "heads_projection_add", "invalidate_casts", "linear", "mlp_fusable", "qkv_projection", "remember_casts"]

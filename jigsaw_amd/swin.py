@@ -27,8 +27,11 @@ from .projection import (
     _GeluMlp,
     _HeadsProjection,
     _QkvProjection,
+    cast_parameters,
+    casts_remembered,
     gelu_mlp,
     heads_projection,
+    heads_projection_add,
     linear,
     mlp_fusable,
     qkv_projection,
@@ -124,15 +127,24 @@ class WindowAttention(nn.Module):
         else:
             self.mask = self.side = None
 
+    def on_grid(self, x: torch.Tensor) -> bool:
+        """Whether the kernel that addresses the windows on the token grid takes these tokens."""
+        return (_compute_dtype(x) == torch.bfloat16 and x.shape[-1] // self.heads == 32 and self.window == 8
+                and x.shape[1] % 8 == 0 and x.shape[2] % 8 == 0)
+
+    def grid_attention(self, x: torch.Tensor, shift: int = 0) -> torch.Tensor:
+        """``(B, h, w, C) -> (B, heads, h * w, 32)`` where :meth:`on_grid`: the kernel addresses the windows on the
+        token grid (rolled by ``-shift``) and forms bias and mask itself: no window partition, no (nW, heads, N, N)
+        bias tensor, no roll."""
+        b, h, w, c = x.shape
+        qkv = qkv_projection(x.to(_compute_dtype(x)).reshape(b, h * w, c), self.qkv.weight, self.qkv.bias, self.heads)
+        return swin_grid_attention_packed(qkv, self.bias_table, self.side, (h, w), shift)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         b, h, w, c = x.shape
         dt = _compute_dtype(x)
-        if dt == torch.bfloat16 and c // self.heads == 32 and self.window == 8 and h % 8 == 0 and w % 8 == 0:
-            # the kernel addresses the windows on the token grid and forms bias and mask itself:
-            # no window partition, no (nW, heads, N, N) bias tensor
-            qkv = qkv_projection(x.to(dt).view(b, h * w, c), self.qkv.weight, self.qkv.bias, self.heads)
-            out = swin_grid_attention_packed(qkv, self.bias_table, self.side, (h, w))
-            return heads_projection(out, self.proj.weight, self.proj.bias).view(b, h, w, c)
+        if self.on_grid(x):
+            return heads_projection(self.grid_attention(x), self.proj.weight, self.proj.bias).view(b, h, w, c)
         x = windows(x, self.window).to(dt)
         n = x.shape[2]
         # the projections write / read the (B, nW, heads, N, d) head layout themselves
@@ -181,19 +193,28 @@ class _WholeBlock(torch.autograd.Function):
         st[5].needs_input_grad = (True,) + pad
         st[6].needs_input_grad = (True, nig[8], nig[9]) + pad
         st[7].needs_input_grad = (True, nig[10], nig[11], nig[12], nig[13], True) + pad
-        roll_args = block._roll_args()
+        params = (qkv_w, qkv_b, proj_w, proj_b, w1, b1, w2, b2)
+        one_cast = not casts_remembered() and all(t.dtype == torch.float32 and t.is_contiguous() for t in params)
+        if one_cast:
+            (qkv_w, proj_w, w1, w2), turned, (qkv_b, proj_b, b1, b2) = cast_parameters(params[::2], params[1::2])
+        roll = block.shift_by and not block.shift_is_local()
         y = _PlainLayerNormFork.forward(st[0], x, n1w, n1b, eps, dt)[0]
-        if block.shift_by:
-            y = _Roll.forward(st[1], y.contiguous(), (-block.shift_by,) * 2, (1, 2), *roll_args)
+        if roll:
+            y = _Roll.forward(st[1], y.contiguous(), (-block.shift_by,) * 2, (1, 2), *block._roll_args())
         qkv = _QkvProjection.forward(st[2], y.view(b, h * w, c), qkv_w, qkv_b, heads)
-        out = _SwinGridAttention.forward(st[3], qkv, table, block.attn.side, (h, w))
-        a = _HeadsProjection.forward(st[4], out, proj_w, proj_b).view(b, h, w, c)
-        if block.shift_by:
-            a = _Roll.forward(st[5], a.contiguous(), (block.shift_by,) * 2, (1, 2), *roll_args)
-        x1 = x + a.to(x.dtype)
+        out = _SwinGridAttention.forward(st[3], qkv, table, block.attn.side, (h, w), 0 if roll else block.shift_by)
+        if roll:
+            a = _HeadsProjection.forward(st[4], out, proj_w, proj_b).view(b, h, w, c)
+            x1 = x + _Roll.forward(st[5], a, (block.shift_by,) * 2, (1, 2), *block._roll_args())
+        else:
+            x1 = _HeadsProjection.forward(st[4], out, proj_w, proj_b, x.contiguous().view(b, h * w, c)).view(b, h, w, c)
         y2 = _PlainLayerNormFork.forward(st[6], x1, n2w, n2b, eps, dt)[0]
         result = _GeluMlp.forward(st[7], y2, w1, b1, w2, b2, x1)
-        ctx.stages, ctx.shifted, ctx.branch_dtype, ctx.grid = st, bool(block.shift_by), a.dtype, (b, h, w, c)
+        if one_cast:  # the gradients are those of the fp32 parameters
+            f32 = torch.float32
+            st[2].dtypes, st[4].dtypes, st[7].dtypes = (f32, f32), (f32, f32), (f32,) * 4
+            st[2].weight_t, st[4].weight_t, st[7].weights_t = turned[0], turned[1], turned[2:]
+        ctx.stages, ctx.rolled, ctx.grid = st, bool(roll), (b, h, w, c)
         return result
 
     @staticmethod
@@ -207,14 +228,12 @@ class _WholeBlock(torch.autograd.Function):
         st, (b, h, w, c) = ctx.stages, ctx.grid
         gy2, gw1, gb1, gw2, gb2, over = _GeluMlp.backward(st[7], grad)
         gx1, gn2w, gn2b = _PlainLayerNormFork.backward(st[6], gy2, over)[:3]
-        ga = gx1.to(ctx.branch_dtype)
-        if ctx.shifted:
-            ga = _Roll.backward(st[5], ga)[0]
+        ga = _Roll.backward(st[5], gx1)[0] if ctx.rolled else gx1
         gout, gpw, gpb = _HeadsProjection.backward(st[4], ga.view(b, h * w, c))[:3]
         dqkv, dtable = _SwinGridAttention.backward(st[3], gout)[:2]
         gy, gqw, gqb = _QkvProjection.backward(st[2], dqkv)[:3]
         gy = gy.view(b, h, w, c)
-        if ctx.shifted:
+        if ctx.rolled:
             gy = _Roll.backward(st[1], gy)[0]
         gx, gn1w, gn1b = _PlainLayerNormFork.backward(st[0], gy, gx1)[:3]
         ctx.stages = None
@@ -279,6 +298,11 @@ class SwinBlock(nn.Module):
         self.attn = WindowAttention(dim, heads, window, tile, shift, groups, device)
         self.norm2 = nn.LayerNorm(dim, eps=eps, device=device)
         self.mlp = nn.Sequential(nn.Linear(dim, 4 * dim, device=device), nn.GELU(), nn.Linear(4 * dim, dim, device=device))
+
+    def shift_is_local(self) -> bool:
+        """Whether the token grid wraps inside this rank: the attention kernel then addresses the shifted windows
+        on the grid as it is and nothing is rolled."""
+        return all(g.size() == 1 for g in self.groups)
 
     def _roll_args(self) -> tuple:
         dist_dims = tuple(d for d, g in zip((1, 2), self.groups) if g.size() > 1)
@@ -357,7 +381,12 @@ class SwinBlock(nn.Module):
                                      attn.proj.weight, attn.proj.bias, self.norm2.weight, self.norm2.bias, fc1.weight, fc1.bias,
                                      fc2.weight, fc2.bias, self)
         y, x = plain_layer_norm_fork(x, self.norm1.weight, self.norm1.bias, self.eps, out_dtype=dt)
-        x = x + self.unshift(self.attn(self.shift(y))).to(x.dtype)
+        if self.attn.on_grid(y) and (not self.shift_by or self.shift_is_local()):
+            b, h, w, c = x.shape
+            x = heads_projection_add(self.attn.grid_attention(y, self.shift_by), self.attn.proj.weight, self.attn.proj.bias,
+                                     x.reshape(b, h * w, c)).view(b, h, w, c)
+        else:
+            x = x + self.unshift(self.attn(self.shift(y))).to(x.dtype)
         y, x = plain_layer_norm_fork(x, self.norm2.weight, self.norm2.bias, self.eps, out_dtype=dt)
         fc1, fc2 = self.mlp[0], self.mlp[2]
         return gelu_mlp(y, fc1.weight, fc1.bias, fc2.weight, fc2.bias, residual=x)

@@ -81,3 +81,39 @@ def test_swin_grid_attention_argument_errors(dev):
         ja.swin_grid_attention(q, q, q, table[:, :1], None, (8, 8))
     with pytest.raises(ValueError):
         ja.swin_grid_attention(q, q, q, table, torch.zeros(1, 64, device=dev), (8, 8))
+
+
+@pytest.mark.parametrize("grid,shift", [((8, 8), 1), ((16, 24), 4), ((24, 8), 7), ((16, 16), 16)])
+def test_windows_of_a_rolled_grid_without_the_roll(grid, shift, dev):
+    """``shift`` addresses the windows of the rolled grid on the grid as it is: output and gradients have the bits of
+    roll, attention, roll back (the table gradient sums the same windows in the same order)."""
+    torch.manual_seed(5)
+    gh, gw = grid
+    b, heads = 2, 3
+    qkv = torch.randn(3, b, heads, gh * gw, 32, device=dev).bfloat16()
+    table = torch.randn(225, heads, device=dev) * 0.5
+    side = js.border_sides(gh, gw, 8, shift, (TileGroup(1, 0), TileGroup(1, 0))).to(torch.uint8).to(dev)
+    g = torch.randn(b, heads, gh * gw, 32, device=dev).bfloat16()
+
+    def rolled(t, by):
+        return torch.roll(t.view(*t.shape[:-2], gh, gw, 32), (by, by), (-3, -2)).reshape(t.shape).contiguous()
+
+    a, ta = qkv.clone().requires_grad_(), table.clone().requires_grad_()
+    out = ja.swin_grid_attention_packed(a, ta, side, grid, shift)
+    da, dta = torch.autograd.grad(out, (a, ta), g)
+    r, tr = rolled(qkv, -shift).requires_grad_(), table.clone().requires_grad_()
+    want = ja.swin_grid_attention_packed(r, tr, side, grid)
+    dr, dtr = torch.autograd.grad(want, (r, tr), rolled(g, -shift))
+    assert torch.equal(out, rolled(want, shift)) and torch.equal(da, rolled(dr, shift)) and torch.equal(dta, dtr)
+
+
+def test_parameters_cast_in_one_launch(dev):
+    """bf16 copies and transposes of fp32 matrices whose edges are no multiples of the 64-wide tiles."""
+    from jigsaw_amd.projection import cast_parameters
+
+    torch.manual_seed(6)
+    ws = [torch.randn(*s, device=dev) for s in ((1, 1), (64, 64), (65, 130), (384, 7))]
+    bs = [torch.randn(n, device=dev) for n in (1, 65, 384)]
+    w, wt, b = cast_parameters(ws, bs)
+    assert all(torch.equal(a, t.bfloat16()) for a, t in zip(w, ws)) and all(torch.equal(a, t.bfloat16()) for a, t in zip(b, bs))
+    assert all(torch.equal(a, t.t().bfloat16()) and a.is_contiguous() for a, t in zip(wt, ws))
