@@ -22,6 +22,7 @@ import ctypes
 import itertools
 import math
 from collections.abc import Sequence
+from functools import lru_cache
 from typing import Any, Protocol
 
 import torch
@@ -393,6 +394,53 @@ def _stuffed(g: torch.Tensor, dense_sp, stride) -> torch.Tensor:
     return up
 
 
+class _Launch:
+    """What a direct launch of one layer on one shape needs, worked out once: the descriptor, the workspace and the
+    shape of the result."""
+
+    __slots__ = ("desc", "nbytes", "shape", "code")
+
+    def __init__(self, desc, nbytes, shape, code) -> None:
+        self.desc, self.nbytes, self.shape, self.code = desc, nbytes, shape, code
+
+
+@lru_cache(maxsize=512)
+def _launch(op: int, dtype: torch.dtype, x_shape, w_shape, stride, padding, dilation, groups: int):
+    """The :class:`_Launch` of a layer with this (padded) input and weight that the C entry points take as it is
+    (op 0 forward, 1 input gradient, 2 weight gradient); ``None`` for the routes that re-shape the layer first and
+    for arguments that do not fit together, which the callers' own checks then name."""
+    n = len(w_shape) - 2
+    if n not in (1, 2, 3) or len(x_shape) != n + 2 or groups < 1 or w_shape[0] % groups or x_shape[1] != w_shape[1] * groups:
+        return None
+    if any(not isinstance(v, (int, tuple)) for v in (stride, padding, dilation)):
+        return None
+    stride, padding, dilation = _tup(stride, n, "stride"), _tup(padding, n, "padding"), _tup(dilation, n, "dilation")
+    if dtype not in _lib._DTYPES or not _single_launch(dtype, x_shape[1], w_shape, stride, padding, dilation, groups):
+        return None
+    out = (x_shape[0], w_shape[0], *_out_spatial(x_shape[2:], w_shape[2:], stride, padding, dilation))
+    desc = _desc(x_shape[0], x_shape[1], w_shape[0], x_shape[2:], w_shape[2:], stride, padding, dilation, groups)
+    nbytes = int(_lib.load().jg_conv_workspace_bytes(desc, op, _lib.dtype_code(dtype)))
+    return _Launch(desc, nbytes, out, _lib.dtype_code(dtype))
+
+
+def _launch_for(op, dtype, x_shape, w_shape, stride, padding, dilation, groups):
+    try:
+        return _launch(op, dtype, tuple(x_shape), tuple(w_shape), stride, padding, dilation, groups)
+    except TypeError:  # lists and the like do not hash: the callers' long way normalises them
+        return None
+
+
+def _scratch(launch: _Launch, device) -> torch.Tensor | None:
+    return torch.empty(launch.nbytes, dtype=torch.uint8, device=device) if launch.nbytes else None
+
+
+def _run_conv_nd(launch: _Launch, x, w, b, y, ws) -> torch.Tensor:
+    rc = _lib.load().jg_conv_fwd(_lib.ptr(y), _lib.ptr(x), _lib.ptr(w), _lib.ptr(b), launch.desc, launch.code, _lib.ptr(ws),
+                                 launch.nbytes, _lib.stream_ptr(x.device))
+    _lib.check(rc, "jg_conv_fwd")
+    return y
+
+
 def _single_launch(dtype, c_in, weight_shape, stride, padding, dilation, groups) -> bool:
     """True where conv_nd / conv_nd_weight hand the tensors to the C entry point as they are (no route that
     re-shapes the layer, copies channel slices or lays out patches first)."""
@@ -418,6 +466,11 @@ def conv_nd(x, w, b=None, *, stride=1, padding=0, dilation=1, groups=1, out=None
     are honoured where the layer runs as one launch on the given tensors and refused on the routes that
     re-shape the layer first."""
     _lib.require_gpu(x, w, b)
+    launch = _launch_for(0, x.dtype, x.shape, w.shape, stride, padding, dilation, groups)
+    if launch is not None and x.dtype == w.dtype and (b is None or b.dtype == x.dtype) and workspace is None:
+        x, w, b = x.contiguous(), w.contiguous(), None if b is None else b.contiguous()
+        y = _out_tensor(out, launch.shape, x.dtype, x.device, "conv_nd")
+        return _run_conv_nd(launch, x, w, b, y, _scratch(launch, x.device))
     if (out is not None or workspace is not None) and not _single_launch(x.dtype, x.shape[1], w.shape, stride, padding, dilation, groups):
         raise NotImplementedError("conv_nd: `out` / `workspace` are taken only where the layer is one launch on the given tensors")
     n = _check_args(x, w, groups, padding)
@@ -464,17 +517,15 @@ def conv_nd(x, w, b=None, *, stride=1, padding=0, dilation=1, groups=1, out=None
     y = _out_tensor(out, (x.shape[0], w.shape[0], *out_sp), x.dtype, x.device, "conv_nd")
     desc = _desc(x.shape[0], x.shape[1], w.shape[0], x.shape[2:], w.shape[2:], stride, padding, dilation, groups)
     ws, nbytes = _workspace(desc, 0, x.dtype, x.device, workspace)
-    rc = _lib.load().jg_conv_fwd(
-        _lib.ptr(y), _lib.ptr(x), _lib.ptr(w), _lib.ptr(b), desc, _lib.dtype_code(x.dtype), _lib.ptr(ws), nbytes,
-        _lib.stream_ptr(x.device),
-    )
-    _lib.check(rc, "jg_conv_fwd")
-    return y
+    return _run_conv_nd(_Launch(desc, nbytes, tuple(y.shape), _lib.dtype_code(x.dtype)), x, w, b, y, ws)
 
 
 def conv_nd_input(input_shape, w, g, *, stride=1, padding=0, dilation=1, groups=1) -> torch.Tensor:
     """``torch.nn.grad.conv{1,2,3}d_input(input_shape, w, g, ...)`` on the HIP kernels."""
     _lib.require_gpu(w, g)
+    launch = _launch_for(1, g.dtype, input_shape, w.shape, stride, padding, dilation, groups)
+    if launch is not None and g.dtype == w.dtype and g.shape == launch.shape:
+        return _run_conv_nd_input(launch, input_shape, w.contiguous(), g.contiguous())
     n = _check_args(g, w, groups, padding)
     input_shape = tuple(int(v) for v in input_shape)
     if len(input_shape) != n + 2:
@@ -535,13 +586,16 @@ def conv_nd_input(input_shape, w, g, *, stride=1, padding=0, dilation=1, groups=
         # gradient of every patch = g_tokens x W, then back to the image layout
         w2t = w.reshape(w.shape[0], -1).t().contiguous()
         return _unpatchify(_proj_nt(_tokens_of(g).contiguous(), w2t, None), input_shape, w.shape[2:], out_sp)
-    gx = torch.empty(input_shape, dtype=g.dtype, device=g.device)
     desc = _desc(input_shape[0], input_shape[1], w.shape[0], input_shape[2:], w.shape[2:], stride, padding, dilation, groups)
-    ws, nbytes = _workspace(desc, 1, g.dtype, g.device)
-    rc = _lib.load().jg_conv_dgrad(
-        _lib.ptr(gx), _lib.ptr(w), _lib.ptr(g), desc, _lib.dtype_code(g.dtype), _lib.ptr(ws), nbytes,
-        _lib.stream_ptr(g.device),
-    )
+    nbytes = int(_lib.load().jg_conv_workspace_bytes(desc, 1, _lib.dtype_code(g.dtype)))
+    return _run_conv_nd_input(_Launch(desc, nbytes, tuple(g.shape), _lib.dtype_code(g.dtype)), input_shape, w, g)
+
+
+def _run_conv_nd_input(launch: _Launch, input_shape, w, g) -> torch.Tensor:
+    gx = torch.empty(input_shape, dtype=g.dtype, device=g.device)
+    ws = _scratch(launch, g.device)
+    rc = _lib.load().jg_conv_dgrad(_lib.ptr(gx), _lib.ptr(w), _lib.ptr(g), launch.desc, launch.code, _lib.ptr(ws), launch.nbytes,
+                                   _lib.stream_ptr(g.device))
     _lib.check(rc, "jg_conv_dgrad")
     return gx
 
@@ -657,10 +711,14 @@ def conv_nd_input_fold(geom: HaloGeometry, w, g, *, stride=1, padding=0, dilatio
             f"grad_output shape {tuple(g.shape)} does not match the convolution of a padded tile {padded} "
             f"(expected {(batch, w.shape[0], *out_sp)})"
         )
-    desc = _desc(batch, c_in, w.shape[0], padded, w.shape[2:], stride, padding, dilation, groups)
-    ws, nbytes = _workspace(desc, 1, g.dtype, g.device, workspace)
+    launch = _launch_for(1, g.dtype, (batch, c_in, *padded), w.shape, stride, padding, dilation, groups) if workspace is None else None
+    if launch is not None:
+        desc, nbytes, ws = launch.desc, launch.nbytes, _scratch(launch, g.device)
+    else:
+        desc = _desc(batch, c_in, w.shape[0], padded, w.shape[2:], stride, padding, dilation, groups)
+        ws, nbytes = _workspace(desc, 1, g.dtype, g.device, workspace)
     lead = (batch, c_in)
-    offs = geom.offsets() if present is None else [tuple(o) for o in present]
+    offs = geom._offsets if present is None else tuple(tuple(o) for o in present)
     if out is None:
         send, tab = new_strips(geom, "pack_bwd", lead, offs, g.dtype, g.device)
         gx = torch.empty(lead + geom.size, dtype=g.dtype, device=g.device)
@@ -690,10 +748,12 @@ def conv_nd_weight(x, weight_shape, g, *, stride=1, padding=0, dilation=1, group
     """
     _lib.require_gpu(x, g)
     weight_shape = tuple(int(v) for v in weight_shape)
+    launch = _launch_for(2, x.dtype, x.shape, weight_shape, stride, padding, dilation, groups)
+    if launch is not None and x.dtype == g.dtype and g.shape == launch.shape and workspace is None:
+        return _run_conv_nd_weight(launch, x.contiguous(), weight_shape, g.contiguous(), with_bias_grad, out, _scratch(launch, x.device))
     n = len(weight_shape) - 2
     if (out is not None or workspace is not None) and not _single_launch(x.dtype, x.shape[1], weight_shape, stride, padding, dilation, groups):
         raise NotImplementedError("conv_nd_weight: `out` / `workspace` are taken only where the layer is one launch on the given tensors")
-    out_w, out_b = (out if with_bias_grad else (out, None)) if out is not None else (None, None)
     if isinstance(padding, str):
         raise NotImplementedError(f"string padding ({padding!r}) is not supported; pass per-axis integers")
     if not isinstance(groups, int) or groups < 1 or weight_shape[0] % groups:
@@ -772,26 +832,28 @@ def conv_nd_weight(x, weight_shape, g, *, stride=1, padding=0, dilation=1, group
                 gb.zero_()
         gw = gw2.reshape(weight_shape)
         return (gw, gb) if with_bias_grad else gw
-    gw = _out_tensor(out_w, weight_shape, x.dtype, x.device, "conv_nd_weight")
     desc = _desc(x.shape[0], x.shape[1], weight_shape[0], x.shape[2:], weight_shape[2:], stride, padding, dilation, groups)
     ws, nbytes = _workspace(desc, 2, x.dtype, x.device, workspace)
+    launch = _Launch(desc, nbytes, tuple(g.shape), _lib.dtype_code(x.dtype))
+    return _run_conv_nd_weight(launch, x, weight_shape, g, with_bias_grad, out, ws)
+
+
+def _run_conv_nd_weight(launch: _Launch, x, weight_shape, g, with_bias_grad, out, ws):
+    out_w, out_b = (out if with_bias_grad else (out, None)) if out is not None else (None, None)
+    gw = _out_tensor(out_w, weight_shape, x.dtype, x.device, "conv_nd_weight")
+    lib, stream = _lib.load(), _lib.stream_ptr(x.device)
     if with_bias_grad:
         # one pass over g for both gradients where the MFMA kernel covers the shape
         gb = _out_tensor(out_b, (weight_shape[0],), x.dtype, x.device, "conv_nd_weight (bias gradient)")
-        rc = _lib.load().jg_conv_wgrad_bias(
-            _lib.ptr(gw), _lib.ptr(gb), _lib.ptr(x), _lib.ptr(g), desc, _lib.dtype_code(x.dtype), _lib.ptr(ws), nbytes,
-            _lib.stream_ptr(x.device),
-        )
+        rc = lib.jg_conv_wgrad_bias(_lib.ptr(gw), _lib.ptr(gb), _lib.ptr(x), _lib.ptr(g), launch.desc, launch.code, _lib.ptr(ws),
+                                    launch.nbytes, stream)
         if rc != -2:
             _lib.check(rc, "jg_conv_wgrad_bias")
             return gw, gb
-    rc = _lib.load().jg_conv_wgrad(
-        _lib.ptr(gw), _lib.ptr(x), _lib.ptr(g), desc, _lib.dtype_code(x.dtype), _lib.ptr(ws), nbytes,
-        _lib.stream_ptr(x.device),
-    )
+    rc = lib.jg_conv_wgrad(_lib.ptr(gw), _lib.ptr(x), _lib.ptr(g), launch.desc, launch.code, _lib.ptr(ws), launch.nbytes, stream)
     _lib.check(rc, "jg_conv_wgrad")
     if with_bias_grad:
-        gb_sep = sum_grad_bias(g, n)
+        gb_sep = sum_grad_bias(g, len(weight_shape) - 2)
         return gw, (gb_sep if out_b is None else out_b.copy_(gb_sep))
     return gw
 
@@ -862,7 +924,8 @@ def _mesh_position(spatial_groups) -> tuple[tuple, tuple]:
     return ranks, sizes
 
 
-def _present_offsets(geom: HaloGeometry, ranks, sizes) -> list:
+@lru_cache(maxsize=256)
+def _present_offsets(geom: HaloGeometry, ranks, sizes) -> tuple:
     out = []
     for o in geom.offsets():
         ok = True
@@ -873,7 +936,7 @@ def _present_offsets(geom: HaloGeometry, ranks, sizes) -> list:
                 ok = False
         if ok:
             out.append(o)
-    return out
+    return tuple(out)
 
 
 def _local_padding(padding, sizes) -> tuple:

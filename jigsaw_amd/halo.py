@@ -15,7 +15,9 @@ from __future__ import annotations
 
 import ctypes
 import itertools
+import math
 from dataclasses import dataclass
+from functools import cached_property, lru_cache
 from typing import Mapping, Sequence
 
 import torch
@@ -145,14 +147,36 @@ class HaloGeometry:
 
     def theirs(self) -> "HaloGeometry":
         """The geometry whose halos are the neighbours' halos of this tile."""
-        if self.same_on_every_rank:
-            return self
+        return self if self.same_on_every_rank else self._theirs
+
+    # What every call on a geometry needs is worked out once per object (:meth:`for_conv` returns the same object
+    # for the same layer and tile): with 26 neighbours the host took longer over it than the kernels over a strip.
+    @cached_property
+    def _theirs(self) -> "HaloGeometry":
         return HaloGeometry(self.size, self.lo if self.their_lo is None else self.their_lo,
                             self.hi if self.their_hi is None else self.their_hi)
 
+    @cached_property
+    def _offsets(self) -> tuple:
+        return tuple(o for o in itertools.product((-1, 0, 1), repeat=self.n_spatial) if any(o))
+
     def offsets(self) -> list:
         """All neighbour offsets except the rank itself."""
-        return [o for o in itertools.product((-1, 0, 1), repeat=self.n_spatial) if any(o)]
+        return list(self._offsets)
+
+    @cached_property
+    def _extents(self) -> dict:
+        """``{verb: ((offset, slot, extent), ...)}`` for the two sizes of strips."""
+        out = {}
+        for verbs, g in ((("assemble", "pack_bwd"), self), (("fold", "pack_fwd"), self.theirs())):
+            three = [(l, n, h) if verbs[0] == "assemble" else (h, n, l) for l, n, h in zip(g.lo, g.size, g.hi)]
+            rows = tuple((o, slot(o), tuple(three[a][v + 1] for a, v in enumerate(o))) for o in self._offsets)
+            out.update({verb: rows for verb in verbs})
+        return out
+
+    @cached_property
+    def _by_offset(self) -> dict:
+        return {verb: {o: extent for o, _, extent in rows} for verb, rows in self._extents.items()}
 
     def strip_extent(self, offset: Sequence[int], verb: str) -> tuple:
         """Spatial extent of the strip of ``offset`` for ``verb``.
@@ -160,16 +184,26 @@ class HaloGeometry:
         ``assemble`` / ``pack_bwd``: (lo, size, hi) for offset (-1, 0, +1);
         ``fold`` / ``pack_fwd``: (their hi, size, their lo).
         """
-        if verb in ("assemble", "pack_bwd"):
-            pick = lambda a, o: (self.lo[a], self.size[a], self.hi[a])[o + 1]  # noqa: E731
-        elif verb in ("fold", "pack_fwd"):
-            t = self.theirs()
-            pick = lambda a, o: (t.hi[a], t.size[a], t.lo[a])[o + 1]  # noqa: E731
-        else:
+        if verb not in self._by_offset:
             raise ValueError(f"unknown verb {verb!r}")
-        return tuple(pick(a, o) for a, o in enumerate(offset))
+        offset = tuple(int(v) for v in offset)
+        if not any(offset):
+            return tuple(self.size)
+        return self._by_offset[verb][offset]
+
+    @cached_property
+    def _c_geoms(self) -> dict:
+        return {}
 
     def c_geom(self, planes: int) -> HaloGeom:
+        g = self._c_geoms.get(planes)
+        if g is None:
+            if len(self._c_geoms) > 64:
+                self._c_geoms.clear()
+            g = self._c_geoms[planes] = self._new_c_geom(planes)
+        return g
+
+    def _new_c_geom(self, planes: int) -> HaloGeom:
         pad = 3 - self.n_spatial
         g = HaloGeom()
         g.planes = planes
@@ -193,6 +227,12 @@ class HaloGeometry:
     ) -> "HaloGeometry":
         """Geometry of a rank's need span; axes with a group of one are not padded
         (the local conv pads them itself, spatial_split.py:75-82)."""
+        return cls._for_conv(tuple(local_in_spatial), tuple(kernel), tuple(stride), tuple(padding), tuple(dilation),
+                             tuple(ranks), tuple(group_sizes))
+
+    @classmethod
+    @lru_cache(maxsize=256)
+    def _for_conv(cls, local_in_spatial, kernel, stride, padding, dilation, ranks, group_sizes) -> "HaloGeometry":
         lo, hi, tlo, thi = [], [], [], []
         for a, n in enumerate(local_in_spatial):
             if group_sizes[a] <= 1:
@@ -209,17 +249,14 @@ class HaloGeometry:
 
 
 def _check_tile(x: torch.Tensor, spatial: tuple, what: str) -> int:
-    ns = len(spatial)
-    if x.dim() < ns + 1:
-        raise ValueError(f"{what}: expected (..., C, {', '.join('S' * ns)}) but got shape {tuple(x.shape)}")
-    if tuple(x.shape[-ns:]) != tuple(spatial):
-        raise ValueError(f"{what}: spatial shape {tuple(x.shape[-ns:])} != expected {tuple(spatial)}")
+    ns, shape = len(spatial), x.shape
+    if len(shape) < ns + 1:
+        raise ValueError(f"{what}: expected (..., C, {', '.join('S' * ns)}) but got shape {tuple(shape)}")
+    if shape[-ns:] != tuple(spatial):
+        raise ValueError(f"{what}: spatial shape {tuple(shape[-ns:])} != expected {tuple(spatial)}")
     if not x.is_contiguous():
         raise ValueError(f"{what}: tensor must be contiguous")
-    planes = 1
-    for s in x.shape[:-ns]:
-        planes *= int(s)
-    return planes
+    return math.prod(shape[:-ns])
 
 
 def _table(
@@ -230,21 +267,21 @@ def _table(
     like: torch.Tensor,
     own: torch.Tensor | None,
 ) -> VoidP27:
-    tab = VoidP27()
-    for o in geom.offsets():
+    at: list = [None] * 27
+    dtype, device = like.dtype, like.device
+    for o, i, extent in geom._extents[verb]:
         t = strips.get(o)
         if t is None:
             continue
-        want = lead + geom.strip_extent(o, verb)
-        if tuple(t.shape) != want:
-            raise ValueError(f"strip {o}: shape {tuple(t.shape)} != expected {want}")
-        if t.dtype != like.dtype or t.device != like.device or not t.is_contiguous():
+        if t.shape != lead + extent:
+            raise ValueError(f"strip {o}: shape {tuple(t.shape)} != expected {lead + extent}")
+        if t.dtype is not dtype or t.device != device or not t.is_contiguous():
             raise ValueError(f"strip {o}: must be contiguous, {like.dtype}, on {like.device}")
         if t.numel():
-            tab[slot(o)] = t.data_ptr()
+            at[i] = t.data_ptr()
     if own is not None:
-        tab[13] = own.data_ptr()
-    return tab
+        at[13] = own.data_ptr()
+    return VoidP27(*at)
 
 
 def halo_assemble(
@@ -291,61 +328,47 @@ def halo_assemble(
     return out
 
 
-_LAYOUTS: dict = {}
-
-
+@lru_cache(maxsize=256)
 def _strip_layout(geom: "HaloGeometry", verb: str, lead: tuple, offs: tuple, elem_size: int) -> tuple:
-    """Where each strip of a pack sits in one flat buffer: ``(offset, shape, strides, start, count)`` per
-    strip in elements, starts rounded up to 256 bytes, and the buffer's length. Cached per geometry."""
-    key = (tuple(geom.size), tuple(geom.lo), tuple(geom.hi), geom.their_lo, geom.their_hi, verb, lead, offs, elem_size)
-    hit = _LAYOUTS.get(key)
-    if hit is not None:
-        return hit
+    """Where the strips of a pack sit in one flat buffer, each from a 256-byte boundary on: ``(pieces, places, start
+    bytes by slot, length in elements)``. ``pieces`` are size-only stand-ins for the strips and the gaps between
+    them, in order (what ``unflatten_dense_tensors`` cuts a buffer by), ``places`` the pieces that are strips."""
     per = 256 // elem_size
-    rows, start = [], 0
+    nothing = torch.empty(1)
+    pieces, places, starts, at = [], [], [None] * 27, 0
     for o in offs:
         shape = lead + geom.strip_extent(o, verb)
-        strides, count = [], 1
-        for n in reversed(shape):
-            strides.append(count)
-            count *= n
-        rows.append((o, shape, tuple(reversed(strides)), start, count))
-        start += (count + per - 1) // per * per
-    if len(_LAYOUTS) > 256:
-        _LAYOUTS.clear()
-    _LAYOUTS[key] = (tuple(rows), start)
-    return _LAYOUTS[key]
+        count = math.prod(shape)
+        places.append(len(pieces))
+        pieces.append(nothing.expand(shape))
+        if count:
+            starts[slot(o)] = at * elem_size
+        gap = -count % per
+        if gap:
+            pieces.append(nothing.expand(gap))
+        at += count + gap
+    return pieces, tuple(places), tuple(starts), at
 
 
 def new_strips(geom: "HaloGeometry", verb: str, lead: tuple, offs: Sequence, dtype: torch.dtype, device) -> tuple:
     """Uninitialised strips for the offsets ``offs`` (``{offset: tensor}``) and the pointer table
     the C entry points take. One allocation holds them all, each strip a contiguous view that
-    starts on a 256-byte boundary: 26 separate allocations cost more host time than the kernels
-    that fill the strips take on the GPU."""
-    elem = torch.empty((), dtype=dtype).element_size()
-    layout, total = _strip_layout(geom, verb, tuple(lead), tuple(offs), elem)
+    starts on a 256-byte boundary, and one call cuts it: 26 separate allocations cost more host time than
+    the kernels that fill the strips take on the GPU."""
+    pieces, places, starts, total = _strip_layout(geom, verb, tuple(lead), tuple(offs), dtype.itemsize)
     flat = torch.empty(total, dtype=dtype, device=device)
     base = flat.data_ptr()
-    out: dict = {}
-    tab = VoidP27()
-    for o, shape, strides, start, count in layout:
-        out[o] = flat.as_strided(shape, strides, start)
-        if count:
-            tab[slot(o)] = base + start * elem
-    return out, tab
+    cut = torch._C._nn.unflatten_dense_tensors(flat, pieces)
+    out = {o: cut[i] for o, i in zip(offs, places)}
+    return out, VoidP27(*[None if s is None else base + s for s in starts])
 
 
 def strip_table(strips: Mapping[Offset, torch.Tensor], geom: "HaloGeometry", verb: str, lead: tuple, like: torch.Tensor) -> VoidP27:
     """The pointer table for strips that exist already (what :func:`new_strips` returned on an earlier
     call), each checked against the shape the geometry gives it."""
-    tab = VoidP27()
-    for o, t in strips.items():
-        want = tuple(lead) + geom.strip_extent(o, verb)
-        if tuple(t.shape) != want or t.dtype != like.dtype or t.device != like.device or not t.is_contiguous():
-            raise ValueError(f"strip {o}: expected a contiguous {like.dtype} tensor of shape {want} on {like.device}")
-        if t.numel():
-            tab[slot(o)] = t.data_ptr()
-    return tab
+    if any(o not in geom._by_offset[verb] for o in strips):
+        raise ValueError(f"offsets {set(strips) - set(geom._offsets)} are no neighbours of this geometry")
+    return _table(strips, geom, verb, tuple(lead), like, None)
 
 
 def halo_pack(
@@ -370,7 +393,7 @@ def halo_pack(
     planes = _check_tile(src, spatial, "halo_pack")
     lead = tuple(src.shape[: -geom.n_spatial])
     verb = "pack_bwd" if from_padded else "pack_fwd"
-    offs = geom.offsets() if present is None else [tuple(o) for o in present]
+    offs = geom._offsets if present is None else tuple(tuple(o) for o in present)
     if out is None:
         out, tab = new_strips(geom, verb, lead, offs, src.dtype, src.device)
     else:
@@ -462,6 +485,12 @@ MAX_AXIS_SEGMENTS = 16
 
 
 def spans_fit_the_strips(local_in_spatial, kernel, stride, padding, dilation, group_sizes) -> bool:
+    """See :func:`_spans_fit` (the answer is kept per layer and tile)."""
+    return _spans_fit(tuple(local_in_spatial), tuple(kernel), tuple(stride), tuple(padding), tuple(dilation), tuple(group_sizes))
+
+
+@lru_cache(maxsize=256)
+def _spans_fit(local_in_spatial, kernel, stride, padding, dilation, group_sizes) -> bool:
     """Whether EVERY rank's need span on every split axis holds its own rows and reaches one tile to
     either side at most: what the one-pass strip functions need. Decided for the whole group, so
     that all of its ranks exchange the same way. ``NotImplementedError`` for an output size the
