@@ -314,9 +314,16 @@ int jg_gn_partial_sqdev(float* sq, const void* x, const float* mean, int64_t bat
                         int64_t channels, int64_t spatial, int64_t groups, int dtype,
                         void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same from ONE pass: mean[n][grp] and sq[n][grp] = sum of (x - mean)^2 of the rank's OWN elements, and
+ * count_sum[n][grp] = their (count, sum), the pair that is added up over the ranks. The centred squares about the
+ * global mean m are sq + count * (mean - m)^2. */
+int jg_gn_moments(float* mean, float* sq, float* count_sum, const void* x, int64_t batch, int64_t channels,
+                  int64_t spatial, int64_t groups, int dtype, void* workspace, size_t workspace_bytes, void* stream);
+
 /* x_norm = (x - mean) * rstd, y = x_norm * weight[c] + bias[c]
  * (_functional.py:370-381). weight / bias (channels,) in `dtype`, either may be
- * NULL. mean / rstd fp32 (batch, groups). */
+ * NULL. mean / rstd fp32 (batch, groups). x_norm NULL: not written (y is computed from x_norm rounded to
+ * `dtype` all the same). */
 int jg_gn_apply(void* y, void* x_norm, const void* x, const float* mean, const float* rstd,
                 const void* weight, const void* bias, int64_t batch, int64_t channels,
                 int64_t spatial, int64_t groups, int dtype, void* stream);
@@ -330,6 +337,25 @@ int jg_gn_partial_bwd(float* gsum, float* gxsum, float* gw, float* gb, const voi
                       const void* x_norm, const void* weight, int64_t batch,
                       int64_t channels, int64_t spatial, int64_t groups, int dtype,
                       void* workspace, size_t workspace_bytes, void* stream);
+
+/* The same from x and the statistics instead of a stored x_norm (which is recomputed in fp32):
+ * sums[n][grp] = (gsum, gxsum); gw / gb in grad_dtype. */
+int jg_gn_partial_bwd_x(float* sums, void* gw, void* gb, const void* g, const void* x, const float* mean,
+                        const float* rstd, const void* weight, int64_t batch, int64_t channels, int64_t spatial,
+                        int64_t groups, int dtype, int grad_dtype, void* workspace, size_t workspace_bytes,
+                        void* stream);
+int jg_gn_bwd_apply_x(void* gx, const void* g, const void* x, const void* weight, const float* mean, const float* rstd,
+                      const float* sums, const float* count, int64_t batch, int64_t channels, int64_t spatial,
+                      int64_t groups, int dtype, void* stream);
+
+/* Forward and backward of a tensor this rank holds whole (no spatial groups): moments + apply, sums + gradient.
+ * gx, gw, gb may be NULL. */
+int jg_gn_forward(void* y, float* mean, float* rstd, const void* x, const void* weight, const void* bias, int64_t batch,
+                  int64_t channels, int64_t spatial, int64_t groups, float eps, int dtype, void* workspace,
+                  size_t workspace_bytes, void* stream);
+int jg_gn_backward(void* gx, void* gw, void* gb, const void* g, const void* x, const float* mean, const float* rstd,
+                   const void* weight, int64_t batch, int64_t channels, int64_t spatial, int64_t groups, int dtype,
+                   int grad_dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 /* gx = rstd * (g * weight[c] - gsum / count - x_norm * gxsum / count) with the
  * COMBINED sums and the global element count per (sample, group), fp32

@@ -5,9 +5,23 @@
 // span. Everything is HBM-bound: 16-byte loads, fp32 accumulation, block partials that a
 // second small kernel adds up in a fixed order (deterministic, no atomics).
 //
+// Passes over the tensor: forward two (the moments of every group from ONE pass, centred on a
+// sample of the block's own elements; normalise + affine), backward two (the sums; the input
+// gradient), both from x and the statistics, x_hat recomputed in fp32 on the way. x_hat itself
+// is only written for a caller that asks for it (jg_gn_apply with x_norm, jg_gn_partial_bwd,
+// jg_gn_bwd_apply): that is one more tensor written and two read, and it is rounded. On
+// 8 x 64 x 1024^2 bf16, 8 groups (1.07 GB a tensor) forward + backward is 1.54 ms = 5.6 TB/s over
+// eight tensors, what a copy reaches; 2.01 ms with three passes forward and x_hat stored. Both
+// passes of a sample before the next one, to find its tensor in the last-level cache, were
+// tried: 1.66 ms (eight launches that are each too small to fill the memory system).
+// Rows and spans start anywhere (S need not be a multiple of 8): a block takes the whole 16-byte
+// words of its range as vectors and the elements before the first and behind the last one by one.
+//
 // Reference behaviour restated here:
 //   jigsaw/modules/normalization/_functional.py:352-385 (forward: sum, centred squares, apply)
 //   jigsaw/modules/normalization/_functional.py:431-468 (backward)
+#include <type_traits>
+
 #include "jg_common.h"
 
 namespace {
@@ -45,35 +59,32 @@ struct alignas(16) Pack {
   typename Elem<DT>::T v[Elem<DT>::VEC];
 };
 
-// Elements [i, i + VEC) of a span of `len` elements; zeros past the end.
 template <int DT>
-__device__ __forceinline__ void load_vec(const typename Elem<DT>::T* p, long long i, long long len, bool vec_ok,
-                                         float out[Elem<DT>::VEC]) {
-  constexpr int V = Elem<DT>::VEC;
-  if (vec_ok && i + V <= len) {
-    const Pack<DT> q = *reinterpret_cast<const Pack<DT>*>(p + i);
+__device__ __forceinline__ void load_vec(const typename Elem<DT>::T* p, float out[Elem<DT>::VEC]) {
+  const Pack<DT> q = *reinterpret_cast<const Pack<DT>*>(p);
 #pragma unroll
-    for (int t = 0; t < V; ++t) out[t] = Elem<DT>::up(q.v[t]);
-  } else {
+  for (int t = 0; t < Elem<DT>::VEC; ++t) out[t] = Elem<DT>::up(q.v[t]);
+}
+template <int DT>
+__device__ __forceinline__ void store_vec(typename Elem<DT>::T* p, const float in[Elem<DT>::VEC]) {
+  Pack<DT> q;
 #pragma unroll
-    for (int t = 0; t < V; ++t) out[t] = (i + t < len) ? Elem<DT>::up(p[i + t]) : 0.0f;
-  }
+  for (int t = 0; t < Elem<DT>::VEC; ++t) q.v[t] = Elem<DT>::down(in[t]);
+  *reinterpret_cast<Pack<DT>*>(p) = q;
 }
 
-template <int DT>
-__device__ __forceinline__ void store_vec(typename Elem<DT>::T* p, long long i, long long len, bool vec_ok,
-                                          const float in[Elem<DT>::VEC]) {
-  constexpr int V = Elem<DT>::VEC;
-  if (vec_ok && i + V <= len) {
-    Pack<DT> q;
-#pragma unroll
-    for (int t = 0; t < V; ++t) q.v[t] = Elem<DT>::down(in[t]);
-    *reinterpret_cast<Pack<DT>*>(p + i) = q;
-  } else {
-#pragma unroll
-    for (int t = 0; t < V; ++t)
-      if (i + t < len) p[i + t] = Elem<DT>::down(in[t]);
-  }
+// The elements [lo, hi) of a tensor over the threads of a block: quad(i, step) for 4 vectors at i, i + step, ..
+// (four loads in flight per thread), vec(i) for one, one(i) for single elements. vec_ok: the tensors start on 16 bytes.
+template <int V, typename QUAD, typename VEC, typename ONE>
+__device__ __forceinline__ void for_range(long long lo, long long hi, bool vec_ok, QUAD quad, VEC vec, ONE one) {
+  long long b0 = (lo + V - 1) / V * V, b1 = hi / V * V;
+  if (!vec_ok || b1 <= b0) b0 = b1 = hi;  // all of it one by one
+  constexpr long long step = (long long)kThreads * V;
+  long long i = b0 + (long long)threadIdx.x * V;
+  for (; i + 3 * step < b1; i += 4 * step) quad(i, step);
+  for (; i < b1; i += step) vec(i);
+  for (long long j = lo + threadIdx.x; j < b0; j += kThreads) one(j);
+  for (long long j = b1 + threadIdx.x; j < hi; j += kThreads) one(j);
 }
 
 // Sum of two per-thread values over the block, fixed order; valid in thread 0.
@@ -96,54 +107,135 @@ __device__ __forceinline__ void block_sum2(float& a, float& b) {
   }
 }
 
+// Chunk b % chunks of unit b / chunks of `len` elements, as absolute element indices.
+__device__ __forceinline__ void chunk_range(unsigned b, long long len, int chunks, long long chunk_len, long long* unit, long long* lo,
+                                            long long* hi) {
+  *unit = b / chunks;
+  const long long from = (b % chunks) * chunk_len;
+  *lo = *unit * len + (from < len ? from : len);
+  *hi = *unit * len + (from + chunk_len < len ? from + chunk_len : len);
+}
+
 // MODE 0: part[0] = sum x                      over a chunk of a (sample, group) span
 // MODE 1: part[0] = sum (x - mean[unit])^2      "
 // MODE 2: part[0] = sum g, part[1] = sum g * y  over a chunk of a (sample, channel) row
-// Block b handles chunk b % chunks of unit b / chunks; partials at part[(b) * 2 + {0, 1}].
+// MODE 3: part[0] = sum g, part[1] = sum g * (y - mean[seg]) * rstd[seg], seg the (sample, group) of the row
+// Partials at part[blockIdx.x * 2 + {0, 1}].
 template <int DT, int MODE>
 __global__ __launch_bounds__(kThreads) void gn_reduce_kernel(float* __restrict__ part,
                                                              const typename Elem<DT>::T* __restrict__ x,
                                                              const typename Elem<DT>::T* __restrict__ y,
-                                                             const float* __restrict__ mean, long long len,
+                                                             const float* __restrict__ mean, const float* __restrict__ rstd,
+                                                             int channels_per_group, long long len,
                                                              int chunks, long long chunk_len, bool vec_ok) {
   constexpr int V = Elem<DT>::VEC;
-  const long long unit = blockIdx.x / chunks;
-  const int chunk = blockIdx.x % chunks;
-  const typename Elem<DT>::T* xs = x + unit * len;
-  const typename Elem<DT>::T* ys = MODE == 2 ? y + unit * len : nullptr;
-  const float m = MODE == 1 ? mean[unit] : 0.0f;
-  const long long lo = chunk * chunk_len;
-  long long hi = lo + chunk_len;
-  if (hi > len) hi = len;
+  long long unit, lo, hi;
+  chunk_range(blockIdx.x, len, chunks, chunk_len, &unit, &lo, &hi);
+  const float m = MODE == 1 ? mean[unit] : MODE == 3 ? mean[unit / channels_per_group] : 0.0f;
   float a = 0.0f, b = 0.0f;
-  for (long long i = lo + (long long)threadIdx.x * V; i < hi; i += (long long)kThreads * V) {
-    float v[V];
-    load_vec<DT>(xs, i, hi, vec_ok, v);
+  auto add = [&](float v, float w) {
     if (MODE == 0) {
-#pragma unroll
-      for (int t = 0; t < V; ++t) a += v[t];
+      a += v;
     } else if (MODE == 1) {
-#pragma unroll
-      for (int t = 0; t < V; ++t) {
-        const float d = (i + t < hi) ? v[t] - m : 0.0f;
-        a += d * d;
-      }
+      const float d = v - m;
+      a += d * d;
     } else {
-      float w[V];
-      load_vec<DT>(ys, i, hi, vec_ok, w);
-#pragma unroll
-      for (int t = 0; t < V; ++t) {
-        a += v[t];
-        b += v[t] * w[t];
-      }
+      a += v;
+      b += v * (MODE == 3 ? w - m : w);
     }
-  }
+  };
+  auto vecs = [&](long long i, long long step, auto count) {
+    float v[count()][V], w[count()][V];
+#pragma unroll
+    for (int q = 0; q < count(); ++q) {
+      load_vec<DT>(x + i + q * step, v[q]);
+      if (MODE >= 2) load_vec<DT>(y + i + q * step, w[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < count(); ++q)
+#pragma unroll
+      for (int t = 0; t < V; ++t) add(v[q][t], MODE >= 2 ? w[q][t] : 0.0f);
+  };
+  for_range<V>(lo, hi, vec_ok, [&](long long i, long long step) { vecs(i, step, std::integral_constant<int, 4>{}); },
+               [&](long long i) { vecs(i, 0, std::integral_constant<int, 1>{}); },
+               [&](long long i) { add(Elem<DT>::up(x[i]), MODE >= 2 ? Elem<DT>::up(y[i]) : 0.0f); });
   block_sum2(a, b);
   if (threadIdx.x == 0) {
     part[(size_t)blockIdx.x * 2 + 0] = a;
-    part[(size_t)blockIdx.x * 2 + 1] = b;
+    part[(size_t)blockIdx.x * 2 + 1] = MODE == 3 ? b * rstd[unit / channels_per_group] : b;
   }
 }
+
+// Moments of a chunk in one pass: part = (mean, sum of squares about it). The sums are centred on the mean of the
+// chunk's first (up to) 256 elements, so that the square of the mean does not swamp the variance.
+template <int DT>
+__global__ __launch_bounds__(kThreads) void gn_moments_kernel(float* __restrict__ part, const typename Elem<DT>::T* __restrict__ x,
+                                                              long long len, int chunks, long long chunk_len, bool vec_ok) {
+  constexpr int V = Elem<DT>::VEC;
+  __shared__ float centre_s;
+  long long unit, lo, hi;
+  chunk_range(blockIdx.x, len, chunks, chunk_len, &unit, &lo, &hi);
+  const long long n = hi - lo;
+  float first = (long long)threadIdx.x < n ? Elem<DT>::up(x[lo + threadIdx.x]) : 0.0f, none = 0.0f;
+  block_sum2(first, none);
+  if (threadIdx.x == 0) centre_s = n > 0 ? first / (float)(n < kThreads ? n : kThreads) : 0.0f;
+  __syncthreads();
+  const float centre = centre_s;
+  float a = 0.0f, b = 0.0f;
+  auto add = [&](float v) {
+    const float d = v - centre;
+    a += d;
+    b += d * d;
+  };
+  auto vecs = [&](long long i, long long step, auto count) {
+    float v[count()][V];
+#pragma unroll
+    for (int q = 0; q < count(); ++q) load_vec<DT>(x + i + q * step, v[q]);
+#pragma unroll
+    for (int q = 0; q < count(); ++q)
+#pragma unroll
+      for (int t = 0; t < V; ++t) add(v[q][t]);
+  };
+  for_range<V>(lo, hi, vec_ok, [&](long long i, long long step) { vecs(i, step, std::integral_constant<int, 4>{}); },
+               [&](long long i) { vecs(i, 0, std::integral_constant<int, 1>{}); }, [&](long long i) { add(Elem<DT>::up(x[i])); });
+  block_sum2(a, b);
+  if (threadIdx.x == 0) {
+    const float shift = n > 0 ? a / (float)n : 0.0f;
+    part[(size_t)blockIdx.x * 2 + 0] = centre + shift;
+    part[(size_t)blockIdx.x * 2 + 1] = n > 0 ? fmaxf(b - a * shift, 0.0f) : 0.0f;
+  }
+}
+
+// The chunks' moments of a unit combined (one wavefront a unit, a lane a chunk, in double): mean, the centred square
+// sum, and what a caller wants of count_sum = (count, sum) pairs and rstd = 1 / sqrt(sq / count + eps).
+__global__ __launch_bounds__(64) void gn_moments_finish_kernel(float* mean, float* sq, float* count_sum, float* rstd,
+                                                               const float* __restrict__ part, long long len, int chunks,
+                                                               long long chunk_len, float eps) {
+  const int u = blockIdx.x, k = threadIdx.x;
+  double n = 0.0, m = 0.0, s = 0.0;
+  if (k < chunks) {
+    const long long from = k * chunk_len;
+    n = (double)(from >= len ? 0 : from + chunk_len < len ? chunk_len : len - from);
+    m = part[((size_t)u * chunks + k) * 2];
+    s = part[((size_t)u * chunks + k) * 2 + 1];
+  }
+  auto total = [](double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+  };
+  const double mu = total(n * m) / (double)len, d = m - mu;
+  const double all = total(s + n * d * d);
+  if (k != 0) return;
+  mean[u] = (float)mu;
+  if (sq != nullptr) sq[u] = (float)all;
+  if (rstd != nullptr) rstd[u] = 1.0f / sqrtf((float)(all / (double)len) + eps);
+  if (count_sum != nullptr) {
+    count_sum[2 * u] = (float)len;
+    count_sum[2 * u + 1] = (float)(mu * (double)len);
+  }
+}
+static_assert(kMaxChunks <= 64, "a lane per chunk");
 
 // out0[u] (and out1[u]) = sum over the chunks of unit u, in chunk order
 __global__ __launch_bounds__(kThreads) void gn_finish_kernel(float* __restrict__ out0, float* __restrict__ out1,
@@ -160,90 +252,119 @@ __global__ __launch_bounds__(kThreads) void gn_finish_kernel(float* __restrict__
   if (out1 != nullptr) out1[u] = b;
 }
 
-// From the row sums a[n][c] = sum g, b[n][c] = sum g * x_norm:
-//   threads [0, N*G):       gsum[n][grp] = sum_c w[c] a[n][c], gxsum[n][grp] = sum_c w[c] b[n][c]
-//   threads [N*G, N*G + C): gb[c] = sum_n a[n][c], gw[c] = sum_n b[n][c]
+__device__ __forceinline__ void store_as(void* p, long long i, float v, int dtype) {
+  if (dtype == JG_F32) static_cast<float*>(p)[i] = v;
+  else if (dtype == JG_BF16) static_cast<uint16_t*>(p)[i] = jg::f32_to_bf16(v);
+  else static_cast<_Float16*>(p)[i] = (_Float16)v;
+}
+
+// From the chunk partials (sum g, sum g * x_norm) of every row (n, c), a wavefront per result, fixed order:
+//   blocks [0, N*G):       sums[n][grp] = (sum_c w[c] sum g, sum_c w[c] sum g * x_norm)
+//   blocks [N*G, N*G + C): gb[c] = sum_n sum g, gw[c] = sum_n sum g * x_norm (dtype `wdtype`)
+// sum0 / sum1: where the two sums of a group go, `stride` floats between groups.
 template <int DT>
-__global__ __launch_bounds__(kThreads) void gn_bwd_finish_kernel(float* __restrict__ gsum, float* __restrict__ gxsum,
-                                                                 float* __restrict__ gw, float* __restrict__ gb,
-                                                                 const float* __restrict__ ra,
-                                                                 const float* __restrict__ rb,
-                                                                 const typename Elem<DT>::T* __restrict__ weight,
-                                                                 long long N, long long C, long long G) {
-  const long long t = (long long)blockIdx.x * kThreads + threadIdx.x;
-  const long long cpg = C / G;
-  if (t < N * G) {
-    const long long n = t / G, grp = t % G;
-    float s0 = 0.0f, s1 = 0.0f;
-    for (long long c = grp * cpg; c < (grp + 1) * cpg; ++c) {
-      const float w = weight != nullptr ? Elem<DT>::up(weight[c]) : 1.0f;
-      s0 += w * ra[n * C + c];
-      s1 += w * rb[n * C + c];
-    }
-    gsum[t] = s0;
-    gxsum[t] = s1;
-  } else if (t < N * G + C) {
-    const long long c = t - N * G;
-    float s0 = 0.0f, s1 = 0.0f;
-    for (long long n = 0; n < N; ++n) {
-      s0 += ra[n * C + c];
-      s1 += rb[n * C + c];
-    }
-    if (gb != nullptr) gb[c] = s0;
-    if (gw != nullptr) gw[c] = s1;
+__global__ __launch_bounds__(64) void gn_bwd_finish_kernel(float* __restrict__ sum0, float* __restrict__ sum1, int stride,
+                                                           void* gw, void* gb, int wdtype, const float* __restrict__ part,
+                                                           const typename Elem<DT>::T* __restrict__ weight, long long N,
+                                                           int C, int G, int chunks) {
+  const int cpg = C / G;
+  const bool group = blockIdx.x < N * G;
+  const long long u = group ? blockIdx.x : blockIdx.x - N * G;
+  const long long items = (group ? cpg : N) * (long long)chunks;  // (row, chunk) pairs of this result
+  float s0 = 0.0f, s1 = 0.0f;
+  for (long long i = threadIdx.x; i < items; i += 64) {
+    const long long r = i / chunks, k = i - r * chunks;
+    const long long row = group ? u * cpg + r : r * C + u;  // rows of a group are consecutive
+    const float w = group && weight != nullptr ? Elem<DT>::up(weight[row % C]) : 1.0f;
+    const float2 v = *reinterpret_cast<const float2*>(part + (row * chunks + k) * 2);
+    s0 += w * v.x;
+    s1 += w * v.y;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    s0 += __shfl_xor(s0, o, 64);
+    s1 += __shfl_xor(s1, o, 64);
+  }
+  if (threadIdx.x != 0) return;
+  if (group) {
+    sum0[u * stride] = s0;
+    sum1[u * stride] = s1;
+  } else {
+    if (gb != nullptr) store_as(gb, u, s0, wdtype);
+    if (gw != nullptr) store_as(gw, u, s1, wdtype);
   }
 }
 
+// What an apply pass reads and writes (a block: chunk b % chunks of row (n, c) = b / chunks)
+struct ApplyArgs {
+  void* out;         // y / gx
+  void* out_norm;    // forward: x_norm, or NULL
+  const void* in;    // x / g
+  const void* in2;   // backward: x_norm (FROM_X: x)
+  const float* mean; // forward and FROM_X
+  const float* rstd;
+  const float* gsum; // backward, `stride` floats between groups
+  const float* gxsum;
+  int stride;
+  const float* cnt;  // backward: elements of every group, or NULL: `count` of each
+  float count;
+  const void* weight;
+  const void* bias;
+  int C, G;
+};
+
 // Forward:  x_norm = (x - mean) * rstd, y = x_norm * w[c] + b[c]
-// Backward: gx = rstd * (g * w[c] - gsum / cnt - x_norm * gxsum / cnt)
-// Block b handles chunk b % chunks of row (n, c) = b / chunks.
-template <int DT, bool BWD>
-__global__ __launch_bounds__(kThreads) void gn_apply_kernel(
-    typename Elem<DT>::T* __restrict__ out, typename Elem<DT>::T* __restrict__ out_norm,
-    const typename Elem<DT>::T* __restrict__ in, const typename Elem<DT>::T* __restrict__ in_norm,
-    const float* __restrict__ s0, const float* __restrict__ s1, const float* __restrict__ s2,
-    const float* __restrict__ cnt, const typename Elem<DT>::T* __restrict__ weight,
-    const typename Elem<DT>::T* __restrict__ bias, long long C, long long G, long long S, int chunks,
-    long long chunk_len, bool vec_ok) {
+// Backward: gx = rstd * (g * w[c] - gsum / cnt - x_norm * gxsum / cnt); FROM_X: x_norm from x as in the forward
+template <int DT, bool BWD, bool FROM_X>
+__global__ __launch_bounds__(kThreads) void gn_apply_kernel(ApplyArgs p, long long S, int chunks, long long chunk_len, bool vec_ok) {
+  typedef typename Elem<DT>::T T;
   constexpr int V = Elem<DT>::VEC;
-  const long long row = blockIdx.x / chunks;
-  const int chunk = blockIdx.x % chunks;
-  const long long n = row / C, c = row % C;
-  const long long seg = n * G + c / (C / G);
-  const float w = weight != nullptr ? Elem<DT>::up(weight[c]) : 1.0f;
-  const float bv = (!BWD && bias != nullptr) ? Elem<DT>::up(bias[c]) : 0.0f;
-  // forward: s0 = mean, s1 = rstd; backward: s0 = rstd, s1 = gsum, s2 = gxsum
-  const float p0 = s0[seg], p1 = s1[seg];
-  const float inv = BWD ? 1.0f / cnt[seg] : 0.0f;
-  const float q1 = BWD ? p1 * inv : 0.0f, q2 = BWD ? s2[seg] * inv : 0.0f;
-  const long long lo = chunk * chunk_len;
-  long long hi = lo + chunk_len;
-  if (hi > S) hi = S;
-  const typename Elem<DT>::T* src = in + row * S;
-  const typename Elem<DT>::T* srcn = BWD ? in_norm + row * S : nullptr;
-  typename Elem<DT>::T* dst = out + row * S;
-  typename Elem<DT>::T* dstn = BWD ? nullptr : out_norm + row * S;
-  for (long long i = lo + (long long)threadIdx.x * V; i < hi; i += (long long)kThreads * V) {
-    float v[V], r[V];
-    load_vec<DT>(src, i, hi, vec_ok, v);
-    if (!BWD) {
-      float xn[V];
+  long long row, lo, hi;
+  // Last block first: the pass before read the tensors from front to back, so that their ends are what the last-level
+  // cache still holds.
+  chunk_range(gridDim.x - 1 - blockIdx.x, S, chunks, chunk_len, &row, &lo, &hi);
+  const int c = (int)(row % p.C);
+  const long long seg = row / p.C * p.G + c / (p.C / p.G);
+  const float w = p.weight != nullptr ? Elem<DT>::up(static_cast<const T*>(p.weight)[c]) : 1.0f;
+  const float bv = (!BWD && p.bias != nullptr) ? Elem<DT>::up(static_cast<const T*>(p.bias)[c]) : 0.0f;
+  const float m = BWD && !FROM_X ? 0.0f : p.mean[seg], rs = p.rstd[seg];
+  const float inv = BWD ? 1.0f / (p.cnt != nullptr ? p.cnt[seg] : p.count) : 0.0f;
+  const float q1 = BWD ? p.gsum[seg * p.stride] * inv : 0.0f, q2 = BWD ? p.gxsum[seg * p.stride] * inv : 0.0f;
+  const T* in = static_cast<const T*>(p.in);
+  const T* in2 = static_cast<const T*>(p.in2);
+  T* out = static_cast<T*>(p.out);
+  T* norm = static_cast<T*>(p.out_norm);
+  // forward: (y, x_norm): x_norm is rounded to the compute dtype and y computed from the rounded value, as the
+  // reference computes y from the x_norm tensor
+  auto forward = [&](float v, float& xn) {
+    xn = Elem<DT>::up(Elem<DT>::down((v - m) * rs));
+    return xn * w + bv;
+  };
+  auto backward = [&](float g, float x) { return rs * (g * w - q1 - (FROM_X ? (x - m) * rs : x) * q2); };
+  auto vecs = [&](long long i, long long step, auto count) {
+    float v[count()][V], x[count()][V];
 #pragma unroll
-      for (int t = 0; t < V; ++t) {
-        // x_norm is stored in the compute dtype and y is computed from the stored value,
-        // as the reference computes y from the x_norm tensor
-        xn[t] = Elem<DT>::up(Elem<DT>::down((v[t] - p0) * p1));
-        r[t] = xn[t] * w + bv;
-      }
-      store_vec<DT>(dstn, i, hi, vec_ok, xn);
-    } else {
-      float xn[V];
-      load_vec<DT>(srcn, i, hi, vec_ok, xn);
-#pragma unroll
-      for (int t = 0; t < V; ++t) r[t] = p0 * (v[t] * w - q1 - xn[t] * q2);
+    for (int q = 0; q < count(); ++q) {
+      load_vec<DT>(in + i + q * step, v[q]);
+      if (BWD) load_vec<DT>(in2 + i + q * step, x[q]);
     }
-    store_vec<DT>(dst, i, hi, vec_ok, r);
-  }
+#pragma unroll
+    for (int q = 0; q < count(); ++q) {
+#pragma unroll
+      for (int t = 0; t < V; ++t) v[q][t] = BWD ? backward(v[q][t], x[q][t]) : forward(v[q][t], x[q][t]);
+      if (!BWD && norm != nullptr) store_vec<DT>(norm + i + q * step, x[q]);
+      store_vec<DT>(out + i + q * step, v[q]);
+    }
+  };
+  for_range<V>(lo, hi, vec_ok, [&](long long i, long long step) { vecs(i, step, std::integral_constant<int, 4>{}); },
+               [&](long long i) { vecs(i, 0, std::integral_constant<int, 1>{}); },
+               [&](long long i) {
+                 const float v = Elem<DT>::up(in[i]);
+                 float xn = BWD ? Elem<DT>::up(in2[i]) : 0.0f;
+                 const float r = BWD ? backward(v, xn) : forward(v, xn);
+                 if (!BWD && norm != nullptr) norm[i] = Elem<DT>::down(xn);
+                 out[i] = Elem<DT>::down(r);
+               });
 }
 
 int chunks_of(long long len) {
@@ -270,24 +391,81 @@ int check(const char* who, int64_t N, int64_t C, int64_t S, int64_t G, int dtype
 }
 
 size_t ws_need(int64_t N, int64_t C, int64_t S) {
-  // the larger of: per-row partials + row sums (backward), per-group partials (forward)
+  // the larger of: per-row partials (backward), per-group partials (forward); and the two sums of every group
   const size_t rows = (size_t)N * (size_t)C;
   return (rows * (size_t)chunks_of(S) * 2 + rows * 2) * sizeof(float) + 256;
 }
 
+// chunk partials of `units` spans of `len` elements into ws
 template <int DT, int MODE>
-int reduce_launch(float* out0, float* out1, const void* x, const void* y, const float* mean, long long units,
-                  long long len, float* ws, hipStream_t s, const char* who) {
+int partials_launch(const void* x, const void* y, const float* mean, const float* rstd, int cpg, long long units,
+                    long long len, float* ws, hipStream_t s, const char* who) {
   typedef typename Elem<DT>::T T;
   if (units == 0) return JG_OK;
   const int chunks = chunks_of(len);
-  const long long cl = chunk_len_of(len, chunks);
-  const bool vec_ok = aligned16(x) && (MODE != 2 || aligned16(y)) && (len * (long long)sizeof(T)) % 16 == 0;
+  const bool vec_ok = aligned16(x) && (MODE < 2 || aligned16(y));
   gn_reduce_kernel<DT, MODE><<<(unsigned)(units * chunks), kThreads, 0, s>>>(
-      ws, static_cast<const T*>(x), static_cast<const T*>(y), mean, len, chunks, cl, vec_ok);
+      ws, static_cast<const T*>(x), static_cast<const T*>(y), mean, rstd, cpg, len, chunks, chunk_len_of(len, chunks), vec_ok);
   JG_CHECK_LAUNCH(who);
-  gn_finish_kernel<<<(unsigned)((units + kThreads - 1) / kThreads), kThreads, 0, s>>>(out0, out1, ws, units, chunks);
+  return JG_OK;
+}
+
+template <int DT, int MODE>
+int reduce_launch(float* out, const void* x, const float* mean, long long units, long long len, float* ws, hipStream_t s,
+                  const char* who) {
+  if (units == 0) return JG_OK;
+  int rc = partials_launch<DT, MODE>(x, nullptr, mean, nullptr, 1, units, len, ws, s, who);
+  if (rc) return rc;
+  gn_finish_kernel<<<(unsigned)((units + kThreads - 1) / kThreads), kThreads, 0, s>>>(out, nullptr, ws, units, chunks_of(len));
   JG_CHECK_LAUNCH(who);
+  return JG_OK;
+}
+
+template <int DT>
+int moments_launch(float* mean, float* sq, float* count_sum, float* rstd, const void* x, long long units, long long len,
+                   float eps, float* ws, hipStream_t s, const char* who) {
+  if (units == 0 || len == 0) return JG_OK;
+  const int chunks = chunks_of(len);
+  const long long cl = chunk_len_of(len, chunks);
+  gn_moments_kernel<DT><<<(unsigned)(units * chunks), kThreads, 0, s>>>(ws, static_cast<const typename Elem<DT>::T*>(x), len,
+                                                                       chunks, cl, aligned16(x));
+  JG_CHECK_LAUNCH(who);
+  gn_moments_finish_kernel<<<(unsigned)units, 64, 0, s>>>(mean, sq, count_sum, rstd, ws, len, chunks, cl, eps);
+  JG_CHECK_LAUNCH(who);
+  return JG_OK;
+}
+
+// The two sums of every (sample, group) and the parameter gradients; mean == NULL: `x` is x_norm.
+template <int DT>
+int bwd_sums_launch(float* sum0, float* sum1, int stride, void* gw, void* gb, int wdtype, const void* g, const void* x,
+                    const float* mean, const float* rstd, const void* weight, long long N, long long C, long long S,
+                    long long G, float* ws, hipStream_t s, const char* who) {
+  if (N * C == 0 || S == 0) return JG_OK;
+  const int cpg = (int)(C / G);
+  const int rc = mean == nullptr ? partials_launch<DT, 2>(g, x, nullptr, nullptr, cpg, N * C, S, ws, s, who)
+                                 : partials_launch<DT, 3>(g, x, mean, rstd, cpg, N * C, S, ws, s, who);
+  if (rc) return rc;
+  gn_bwd_finish_kernel<DT><<<(unsigned)(N * G + C), 64, 0, s>>>(sum0, sum1, stride, gw, gb, wdtype, ws,
+                                                                static_cast<const typename Elem<DT>::T*>(weight), N, (int)C,
+                                                                (int)G, chunks_of(S));
+  JG_CHECK_LAUNCH(who);
+  return JG_OK;
+}
+
+template <int DT, bool BWD, bool FROM_X>
+int apply_launch(const ApplyArgs& a, long long N, long long S, hipStream_t s, const char* who) {
+  const long long rows = N * a.C;
+  if (rows == 0 || S == 0) return JG_OK;
+  const int chunks = chunks_of(S);
+  const bool vec_ok = aligned16(a.out) && aligned16(a.in) && aligned16(a.in2) && aligned16(a.out_norm);
+  gn_apply_kernel<DT, BWD, FROM_X><<<(unsigned)(rows * chunks), kThreads, 0, s>>>(a, S, chunks, chunk_len_of(S, chunks), vec_ok);
+  JG_CHECK_LAUNCH(who);
+  return JG_OK;
+}
+
+int check_ws(const char* who, const void* ws, size_t bytes, int64_t batch, int64_t channels, int64_t spatial) {
+  const size_t need = batch <= 0 || channels <= 0 || spatial <= 0 ? 256 : ws_need(batch, channels, spatial);
+  if (ws == nullptr || bytes < need) JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, bytes, need);
   return JG_OK;
 }
 
@@ -312,12 +490,10 @@ extern "C" int jg_gn_partial_sum(float* sum, const void* x, int64_t batch, int64
   int rc = check(who, batch, channels, spatial, groups, dtype);
   if (rc) return rc;
   JG_REQUIRE(sum && x, "%s: NULL pointer", who);
-  if (workspace == nullptr || workspace_bytes < jg_gn_workspace_bytes(batch, channels, spatial))
-    JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, workspace_bytes,
-            jg_gn_workspace_bytes(batch, channels, spatial));
+  if ((rc = check_ws(who, workspace, workspace_bytes, batch, channels, spatial))) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const long long units = batch * groups, len = channels / groups * spatial;
-#define CALL(DT) reduce_launch<DT, 0>(sum, nullptr, x, nullptr, nullptr, units, len, static_cast<float*>(workspace), s, who)
+#define CALL(DT) reduce_launch<DT, 0>(sum, x, nullptr, units, len, static_cast<float*>(workspace), s, who)
   JG_GN_DISPATCH(CALL)
 #undef CALL
 }
@@ -329,35 +505,28 @@ extern "C" int jg_gn_partial_sqdev(float* sq, const void* x, const float* mean, 
   int rc = check(who, batch, channels, spatial, groups, dtype);
   if (rc) return rc;
   JG_REQUIRE(sq && x && mean, "%s: NULL pointer", who);
-  if (workspace == nullptr || workspace_bytes < jg_gn_workspace_bytes(batch, channels, spatial))
-    JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, workspace_bytes,
-            jg_gn_workspace_bytes(batch, channels, spatial));
+  if ((rc = check_ws(who, workspace, workspace_bytes, batch, channels, spatial))) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const long long units = batch * groups, len = channels / groups * spatial;
-#define CALL(DT) reduce_launch<DT, 1>(sq, nullptr, x, nullptr, mean, units, len, static_cast<float*>(workspace), s, who)
+#define CALL(DT) reduce_launch<DT, 1>(sq, x, mean, units, len, static_cast<float*>(workspace), s, who)
   JG_GN_DISPATCH(CALL)
 #undef CALL
 }
 
-namespace {
-template <int DT, bool BWD>
-int apply_launch(void* out, void* out_norm, const void* in, const void* in_norm, const float* s0, const float* s1,
-                 const float* s2, const float* cnt, const void* weight, const void* bias, long long N,
-                 long long C, long long S, long long G, hipStream_t s, const char* who) {
-  typedef typename Elem<DT>::T T;
-  const long long rows = N * C;
-  if (rows == 0 || S == 0) return JG_OK;
-  const int chunks = chunks_of(S);
-  const long long cl = chunk_len_of(S, chunks);
-  const bool vec_ok = aligned16(out) && aligned16(in) && (BWD ? aligned16(in_norm) : aligned16(out_norm)) &&
-                      (S * (long long)sizeof(T)) % 16 == 0;
-  gn_apply_kernel<DT, BWD><<<(unsigned)(rows * chunks), kThreads, 0, s>>>(
-      static_cast<T*>(out), static_cast<T*>(out_norm), static_cast<const T*>(in), static_cast<const T*>(in_norm), s0,
-      s1, s2, cnt, static_cast<const T*>(weight), static_cast<const T*>(bias), C, G, S, chunks, cl, vec_ok);
-  JG_CHECK_LAUNCH(who);
-  return JG_OK;
+extern "C" int jg_gn_moments(float* mean, float* sq, float* count_sum, const void* x, int64_t batch, int64_t channels,
+                             int64_t spatial, int64_t groups, int dtype, void* workspace, size_t workspace_bytes,
+                             void* stream) {
+  const char* who = "jg_gn_moments";
+  int rc = check(who, batch, channels, spatial, groups, dtype);
+  if (rc) return rc;
+  JG_REQUIRE(mean && sq && count_sum && x, "%s: NULL pointer", who);
+  if ((rc = check_ws(who, workspace, workspace_bytes, batch, channels, spatial))) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const long long units = batch * groups, len = channels / groups * spatial;
+#define CALL(DT) moments_launch<DT>(mean, sq, count_sum, nullptr, x, units, len, 0.0f, static_cast<float*>(workspace), s, who)
+  JG_GN_DISPATCH(CALL)
+#undef CALL
 }
-}  // namespace
 
 extern "C" int jg_gn_apply(void* y, void* x_norm, const void* x, const float* mean, const float* rstd,
                            const void* weight, const void* bias, int64_t batch, int64_t channels,
@@ -365,10 +534,102 @@ extern "C" int jg_gn_apply(void* y, void* x_norm, const void* x, const float* me
   const char* who = "jg_gn_apply";
   int rc = check(who, batch, channels, spatial, groups, dtype);
   if (rc) return rc;
-  JG_REQUIRE(y && x_norm && x && mean && rstd, "%s: NULL pointer", who);
+  JG_REQUIRE(y && x && mean && rstd, "%s: NULL pointer", who);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define CALL(DT) \
-  apply_launch<DT, false>(y, x_norm, x, nullptr, mean, rstd, nullptr, nullptr, weight, bias, batch, channels, spatial, groups, s, who)
+  ApplyArgs a = {};
+  a.out = y; a.out_norm = x_norm; a.in = x; a.mean = mean; a.rstd = rstd; a.weight = weight; a.bias = bias;
+  a.C = (int)channels; a.G = (int)groups;
+#define CALL(DT) apply_launch<DT, false, true>(a, batch, spatial, s, who)
+  JG_GN_DISPATCH(CALL)
+#undef CALL
+}
+
+// Both passes of the forward / of the backward for a tensor that one rank holds whole.
+namespace {
+template <int DT>
+int forward_all(void* y, float* mean, float* rstd, const void* x, const void* weight, const void* bias, long long N,
+                long long C, long long S, long long G, float eps, float* ws, hipStream_t s, const char* who) {
+  int rc = moments_launch<DT>(mean, nullptr, nullptr, rstd, x, N * G, C / G * S, eps, ws, s, who);
+  if (rc) return rc;
+  ApplyArgs a = {};
+  a.out = y; a.in = x; a.mean = mean; a.rstd = rstd; a.weight = weight; a.bias = bias; a.C = (int)C; a.G = (int)G;
+  return apply_launch<DT, false, true>(a, N, S, s, who);
+}
+
+template <int DT>
+int backward_all(void* gx, void* gw, void* gb, int wdtype, const void* g, const void* x, const float* mean, const float* rstd,
+                 const void* weight, long long N, long long C, long long S, long long G, float* ws, hipStream_t s, const char* who) {
+  const long long rows = N * C;
+  float* sums = ws + (size_t)rows * chunks_of(S) * 2;
+  int rc = bwd_sums_launch<DT>(sums, sums + 1, 2, gw, gb, wdtype, g, x, mean, rstd, weight, N, C, S, G, ws, s, who);
+  if (rc || gx == nullptr) return rc;
+  ApplyArgs a = {};
+  a.out = gx; a.in = g; a.in2 = x; a.mean = mean; a.rstd = rstd; a.gsum = sums; a.gxsum = sums + 1; a.stride = 2;
+  a.count = (float)(C / G * S);
+  a.weight = weight; a.C = (int)C; a.G = (int)G;
+  return apply_launch<DT, true, true>(a, N, S, s, who);
+}
+}  // namespace
+
+extern "C" int jg_gn_forward(void* y, float* mean, float* rstd, const void* x, const void* weight, const void* bias,
+                             int64_t batch, int64_t channels, int64_t spatial, int64_t groups, float eps, int dtype,
+                             void* workspace, size_t workspace_bytes, void* stream) {
+  const char* who = "jg_gn_forward";
+  int rc = check(who, batch, channels, spatial, groups, dtype);
+  if (rc) return rc;
+  JG_REQUIRE(y && mean && rstd && x, "%s: NULL pointer", who);
+  if ((rc = check_ws(who, workspace, workspace_bytes, batch, channels, spatial))) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define CALL(DT) forward_all<DT>(y, mean, rstd, x, weight, bias, batch, channels, spatial, groups, eps, static_cast<float*>(workspace), s, who)
+  JG_GN_DISPATCH(CALL)
+#undef CALL
+}
+
+extern "C" int jg_gn_backward(void* gx, void* gw, void* gb, const void* g, const void* x, const float* mean,
+                              const float* rstd, const void* weight, int64_t batch, int64_t channels, int64_t spatial,
+                              int64_t groups, int dtype, int grad_dtype, void* workspace, size_t workspace_bytes,
+                              void* stream) {
+  const char* who = "jg_gn_backward";
+  int rc = check(who, batch, channels, spatial, groups, dtype);
+  if (rc) return rc;
+  JG_REQUIRE(jg::dtype_size(grad_dtype) != 0, "%s: unknown gradient dtype %d", who, grad_dtype);
+  JG_REQUIRE(g && x && mean && rstd, "%s: NULL pointer", who);
+  if ((rc = check_ws(who, workspace, workspace_bytes, batch, channels, spatial))) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define CALL(DT) backward_all<DT>(gx, gw, gb, grad_dtype, g, x, mean, rstd, weight, batch, channels, spatial, groups, static_cast<float*>(workspace), s, who)
+  JG_GN_DISPATCH(CALL)
+#undef CALL
+}
+
+// The pieces of the backward of a sharded tensor, from x_norm (mean NULL) or from x.
+extern "C" int jg_gn_partial_bwd_x(float* sums, void* gw, void* gb, const void* g, const void* x, const float* mean,
+                                   const float* rstd, const void* weight, int64_t batch, int64_t channels, int64_t spatial,
+                                   int64_t groups, int dtype, int grad_dtype, void* workspace, size_t workspace_bytes,
+                                   void* stream) {
+  const char* who = "jg_gn_partial_bwd_x";
+  int rc = check(who, batch, channels, spatial, groups, dtype);
+  if (rc) return rc;
+  JG_REQUIRE(jg::dtype_size(grad_dtype) != 0, "%s: unknown gradient dtype %d", who, grad_dtype);
+  JG_REQUIRE(sums && g && x && mean && rstd, "%s: NULL pointer", who);
+  if ((rc = check_ws(who, workspace, workspace_bytes, batch, channels, spatial))) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define CALL(DT) bwd_sums_launch<DT>(sums, sums + 1, 2, gw, gb, grad_dtype, g, x, mean, rstd, weight, batch, channels, spatial, groups, static_cast<float*>(workspace), s, who)
+  JG_GN_DISPATCH(CALL)
+#undef CALL
+}
+
+extern "C" int jg_gn_bwd_apply_x(void* gx, const void* g, const void* x, const void* weight, const float* mean,
+                                 const float* rstd, const float* sums, const float* count, int64_t batch, int64_t channels,
+                                 int64_t spatial, int64_t groups, int dtype, void* stream) {
+  const char* who = "jg_gn_bwd_apply_x";
+  int rc = check(who, batch, channels, spatial, groups, dtype);
+  if (rc) return rc;
+  JG_REQUIRE(gx && g && x && mean && rstd && sums && count, "%s: NULL pointer", who);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  ApplyArgs a = {};
+  a.out = gx; a.in = g; a.in2 = x; a.mean = mean; a.rstd = rstd; a.gsum = sums; a.gxsum = sums + 1; a.stride = 2;
+  a.cnt = count; a.weight = weight; a.C = (int)channels; a.G = (int)groups;
+#define CALL(DT) apply_launch<DT, true, true>(a, batch, spatial, s, who)
   JG_GN_DISPATCH(CALL)
 #undef CALL
 }
@@ -381,26 +642,9 @@ extern "C" int jg_gn_partial_bwd(float* gsum, float* gxsum, float* gw, float* gb
   int rc = check(who, batch, channels, spatial, groups, dtype);
   if (rc) return rc;
   JG_REQUIRE(gsum && gxsum && g && x_norm, "%s: NULL pointer", who);
-  if (workspace == nullptr || workspace_bytes < jg_gn_workspace_bytes(batch, channels, spatial))
-    JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, workspace_bytes,
-            jg_gn_workspace_bytes(batch, channels, spatial));
+  if ((rc = check_ws(who, workspace, workspace_bytes, batch, channels, spatial))) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const long long rows = batch * channels;
-  if (rows == 0) return JG_OK;
-  float* part = static_cast<float*>(workspace);
-  float* ra = part + (size_t)rows * chunks_of(spatial) * 2;  // row sums behind the chunk partials
-  float* rb = ra + rows;
-  const unsigned fin = (unsigned)((batch * groups + channels + kThreads - 1) / kThreads);
-#define CALL(DT)                                                                                          \
-  [&]() -> int {                                                                                          \
-    int r2 = reduce_launch<DT, 2>(ra, rb, g, x_norm, nullptr, rows, spatial, part, s, who);               \
-    if (r2) return r2;                                                                                    \
-    gn_bwd_finish_kernel<DT><<<fin, kThreads, 0, s>>>(gsum, gxsum, gw, gb, ra, rb,                        \
-                                                      static_cast<const Elem<DT>::T*>(weight), batch,     \
-                                                      channels, groups);                                  \
-    JG_CHECK_LAUNCH(who);                                                                                 \
-    return JG_OK;                                                                                         \
-  }()
+#define CALL(DT) bwd_sums_launch<DT>(gsum, gxsum, 1, gw, gb, JG_F32, g, x_norm, nullptr, nullptr, weight, batch, channels, spatial, groups, static_cast<float*>(workspace), s, who)
   JG_GN_DISPATCH(CALL)
 #undef CALL
 }
@@ -413,8 +657,10 @@ extern "C" int jg_gn_bwd_apply(void* gx, const void* g, const void* x_norm, cons
   if (rc) return rc;
   JG_REQUIRE(gx && g && x_norm && rstd && gsum && gxsum && count, "%s: NULL pointer", who);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define CALL(DT) \
-  apply_launch<DT, true>(gx, nullptr, g, x_norm, rstd, gsum, gxsum, count, weight, nullptr, batch, channels, spatial, groups, s, who)
+  ApplyArgs a = {};
+  a.out = gx; a.in = g; a.in2 = x_norm; a.rstd = rstd; a.gsum = gsum; a.gxsum = gxsum; a.stride = 1;
+  a.cnt = count; a.weight = weight; a.C = (int)channels; a.G = (int)groups;
+#define CALL(DT) apply_launch<DT, true, false>(a, batch, spatial, s, who)
   JG_GN_DISPATCH(CALL)
 #undef CALL
 }

@@ -81,6 +81,26 @@ def partial_sqdev(x: torch.Tensor, mean: torch.Tensor, num_groups: int) -> torch
     return out
 
 
+def _global_statistics(x: torch.Tensor, num_groups: int, spatial_groups, eps: float) -> tuple:
+    """``(mean, rstd, count)`` over every rank's positions, fp32 ``(N, num_groups)``: the rank's own moments from one
+    pass over ``x``, then one collective for (count, sum) and one for the squares about the global mean."""
+    n, c, s = _dims(x)
+    lib, dev = _lib.load(), x.device
+    local_mean = torch.empty(n, num_groups, dtype=torch.float32, device=dev)
+    var = torch.empty_like(local_mean)
+    stats = torch.empty(n, num_groups, 2, dtype=torch.float32, device=dev)
+    ws, nbytes = _workspace(lib, n, c, s, dev)
+    rc = lib.jg_gn_moments(_lib.ptr(local_mean), _lib.ptr(var), _lib.ptr(stats), _lib.ptr(x), n, c, s, num_groups,
+                           _lib.dtype_code(x.dtype), _lib.ptr(ws), nbytes, _lib.stream_ptr(dev))
+    _lib.check(rc, "jg_gn_moments")
+    _all_reduce_sum(stats, spatial_groups)
+    count, total = stats.unbind(dim=-1)
+    mean = total / count
+    var = torch.addcmul(var, float(c // num_groups * s) * (local_mean - mean), local_mean - mean)
+    _all_reduce_sum(var, spatial_groups)
+    return mean.contiguous(), torch.rsqrt(var / count + eps).contiguous(), count.contiguous()
+
+
 class _GroupNorm(torch.autograd.Function):
     """Autograd function of the GroupNorm over a spatially sharded input (HIP kernels inside)."""
 
@@ -97,17 +117,7 @@ class _GroupNorm(torch.autograd.Function):
         lib = _lib.load()
         dev = x.device
 
-        # global count and sum per (sample, group) in one collective per process group
-        local = partial_sum(x, num_groups)
-        stats = torch.stack([torch.full_like(local, float(c // num_groups * s)), local], dim=-1)
-        _all_reduce_sum(stats, spatial_groups)
-        count, total = stats.unbind(dim=-1)
-        mean = (total / count).contiguous()
-        # centred on the global mean before squaring (two-pass variance)
-        var = partial_sqdev(x, mean, num_groups)
-        _all_reduce_sum(var, spatial_groups)
-        rstd = torch.rsqrt(var / count + eps).contiguous()
-
+        mean, rstd, count = _global_statistics(x, num_groups, spatial_groups, eps)
         y = torch.empty_like(x)
         x_norm = torch.empty_like(x)
         rc = lib.jg_gn_apply(_lib.ptr(y), _lib.ptr(x_norm), _lib.ptr(x), _lib.ptr(mean), _lib.ptr(rstd),
@@ -115,7 +125,6 @@ class _GroupNorm(torch.autograd.Function):
                              _lib.stream_ptr(dev))
         _lib.check(rc, "jg_gn_apply")
 
-        count = count.contiguous()
         ctx.num_groups = num_groups
         ctx.spatial_groups = spatial_groups
         ctx.has_weight, ctx.has_bias = weight is not None, bias is not None
@@ -166,9 +175,84 @@ class _GroupNorm(torch.autograd.Function):
         return (grad_x, None, gw.to(dt_w) if need_w else None, gb.to(dt_b) if need_b else None, None, None)
 
 
+class _GroupNormOutput(torch.autograd.Function):
+    """``_GroupNorm`` for a caller that wants ``y`` alone: ``x`` and the statistics are kept for the backward instead of
+    ``x_norm``, which is then neither written nor read (the backward recomputes it, unrounded, on the way)."""
+
+    @staticmethod
+    def forward(ctx, x, num_groups, weight, bias, spatial_groups, eps):  # noqa: D102
+        cdt = _compute_dtype(x)
+        x = x.to(cdt).contiguous()
+        w = None if weight is None else weight.to(cdt).contiguous()
+        b = None if bias is None else bias.to(cdt).contiguous()
+        n, c, s = _dims(x)
+        lib, dev, code = _lib.load(), x.device, _lib.dtype_code(cdt)
+        y = torch.empty_like(x)
+        if spatial_groups:
+            mean, rstd, count = _global_statistics(x, num_groups, spatial_groups, eps)
+            rc = lib.jg_gn_apply(_lib.ptr(y), None, _lib.ptr(x), _lib.ptr(mean), _lib.ptr(rstd), _lib.ptr(w), _lib.ptr(b),
+                                 n, c, s, num_groups, code, _lib.stream_ptr(dev))
+            _lib.check(rc, "jg_gn_apply")
+        else:
+            mean, rstd = torch.empty(2, n, num_groups, dtype=torch.float32, device=dev).unbind(0)
+            count = None
+            ws, nbytes = _workspace(lib, n, c, s, dev)
+            rc = lib.jg_gn_forward(_lib.ptr(y), _lib.ptr(mean), _lib.ptr(rstd), _lib.ptr(x), _lib.ptr(w), _lib.ptr(b), n, c, s,
+                                   num_groups, float(eps), code, _lib.ptr(ws), nbytes, _lib.stream_ptr(dev))
+            _lib.check(rc, "jg_gn_forward")
+        ctx.num_groups, ctx.spatial_groups = num_groups, spatial_groups
+        ctx.dtypes = (None if weight is None else weight.dtype, None if bias is None else bias.dtype)
+        ctx.save_for_backward(x, mean, rstd, count, w)
+        return y
+
+    @staticmethod
+    def backward(ctx, grad_output):  # noqa: D102
+        x, mean, rstd, count, w = ctx.saved_tensors
+        g = grad_output.to(x.dtype).contiguous()
+        n, c, s = _dims(x)
+        groups = ctx.num_groups
+        lib, dev, code, stream = _lib.load(), g.device, _lib.dtype_code(x.dtype), _lib.stream_ptr(g.device)
+        need_x = ctx.needs_input_grad[0]
+        dt_w, dt_b = ctx.dtypes
+        need_w = dt_w is not None and ctx.needs_input_grad[2]
+        need_b = dt_b is not None and ctx.needs_input_grad[3]
+        # both parameter gradients leave the kernel in one dtype: theirs where they agree
+        gdt = next((d for d in (dt_w, dt_b) if d in _lib._DTYPES), torch.float32)
+        if dt_w is not None and dt_b is not None and dt_w != dt_b:
+            gdt = torch.float32
+        gw = torch.empty(c, dtype=gdt, device=dev) if need_w else None
+        gb = torch.empty(c, dtype=gdt, device=dev) if need_b else None
+        gx = torch.empty_like(g) if need_x else None
+        ws, nbytes = _workspace(lib, n, c, s, dev)
+        if not ctx.spatial_groups:
+            rc = lib.jg_gn_backward(_lib.ptr(gx), _lib.ptr(gw), _lib.ptr(gb), _lib.ptr(g), _lib.ptr(x), _lib.ptr(mean),
+                                    _lib.ptr(rstd), _lib.ptr(w), n, c, s, groups, code, _lib.dtype_code(gdt), _lib.ptr(ws), nbytes,
+                                    stream)
+            _lib.check(rc, "jg_gn_backward")
+        else:
+            sums = torch.empty(n, groups, 2, dtype=torch.float32, device=dev)
+            rc = lib.jg_gn_partial_bwd_x(_lib.ptr(sums), _lib.ptr(gw), _lib.ptr(gb), _lib.ptr(g), _lib.ptr(x), _lib.ptr(mean),
+                                         _lib.ptr(rstd), _lib.ptr(w), n, c, s, groups, code, _lib.dtype_code(gdt), _lib.ptr(ws),
+                                         nbytes, stream)
+            _lib.check(rc, "jg_gn_partial_bwd_x")
+            if need_x:
+                _all_reduce_sum(sums, ctx.spatial_groups)
+                rc = lib.jg_gn_bwd_apply_x(_lib.ptr(gx), _lib.ptr(g), _lib.ptr(x), _lib.ptr(w), _lib.ptr(mean), _lib.ptr(rstd),
+                                           _lib.ptr(sums), _lib.ptr(count), n, c, s, groups, code, stream)
+                _lib.check(rc, "jg_gn_bwd_apply_x")
+        return gx, None, None if gw is None else gw.to(dt_w), None if gb is None else gb.to(dt_b), None, None
+
+
 def group_norm(x, num_groups, weight=None, bias=None, spatial_groups=(), eps=1e-5):
-    """``_GroupNorm.apply(...)[0]``, the call of ``DistributedGroupNorm.forward``."""
-    return _GroupNorm.apply(x, num_groups, weight, bias, spatial_groups, eps)[0]
+    """``_GroupNorm.apply(...)[0]``, the call of ``DistributedGroupNorm.forward``, without the tensors only its other
+    results need."""
+    _lib.require_gpu(x, weight, bias)
+    if x.shape[1] % num_groups != 0:
+        raise ValueError(f"{x.shape[1]} channels do not divide into {num_groups} groups")
+    if x.numel() == 0:
+        return _GroupNorm.apply(x, num_groups, weight, bias, spatial_groups, eps)[0]
+    split = tuple(g for g in spatial_groups or () if g is not None and int(g.size()) > 1)
+    return _GroupNormOutput.apply(x, num_groups, weight, bias, split, eps)
 
 
 __all__ = ["_GroupNorm", "group_norm", "partial_sqdev", "partial_sum"]

@@ -7,6 +7,8 @@ of a shard see the other shards' contributions through a stand-in group that hol
 Tolerances: rel-L2 <= 1e-5 in fp32, 2e-2 in bf16.
 """
 
+import math
+
 import pytest
 import torch
 
@@ -122,3 +124,62 @@ def test_groupnorm_argument_errors(dev):
     x = torch.zeros(1, 6, 4, 4, device=dev)
     with pytest.raises(ValueError):
         jgn.group_norm(x, 4)
+
+
+@pytest.mark.parametrize("case", CASES + [
+    ((1, 4, 1, 1), 2, torch.bfloat16, True, True, 1), ((2, 6, 3, 7), 2, torch.bfloat16, True, True, 1),
+    ((3, 8, 1, 257), 4, torch.float16, True, False, 1), ((2, 4, 513, 130), 2, torch.bfloat16, False, False, 1),
+    ((40, 8, 640, 650), 4, torch.bfloat16, True, True, 1),
+], ids=str)
+def test_group_norm_without_x_norm(case, dev):
+    """``group_norm`` (statistics from one pass, x_hat recomputed in the backward) whole and sharded: rows that start off
+    the 16-byte grid, spans of one element, spans of many chunks, a mean far above the spread, more samples than one
+    step of the last-level cache takes."""
+    shape, G, dtype, has_w, has_b, P = case
+    torch.manual_seed(9)
+    big = math.prod(shape) > 1 << 24
+    x = (torch.randn(*shape, device=dev) * 0.5 + (0.3 if dtype != torch.float32 else 40.0)).to(dtype)
+    w = (1 + 0.2 * torch.randn(shape[1], device=dev)).to(dtype) if has_w else None
+    b = (0.2 * torch.randn(shape[1], device=dev)).to(dtype) if has_b else None
+    g = torch.randn(*shape, device=dev).to(dtype)
+    ref = torch.float32 if big else torch.float64
+    leaves = [None if t is None else t.to(ref).requires_grad_() for t in (x, w, b)]
+    affine = [torch.ones(shape[1], device=dev, dtype=ref) if leaves[1] is None else leaves[1], leaves[2]]  # torch's own backward wants a weight
+    want = torch.nn.functional.group_norm(leaves[0], G, *affine, 1e-5)
+    grads = torch.autograd.grad(want, [t for t in leaves if t is not None], g.to(ref))
+    tol = max(TOL[dtype], 2e-5)
+    got_leaves = [None if t is None else t.clone().requires_grad_() for t in (x, w, b)]
+    y = jgn.group_norm(got_leaves[0], G, got_leaves[1], got_leaves[2])
+    got = torch.autograd.grad(y, [t for t in got_leaves if t is not None], g)
+    assert y.dtype == dtype and rel_l2(y, want) < tol
+    for a, r in zip(got, grads):
+        assert a.dtype == dtype and (rel_l2(a, r) < tol or r.norm() < 1e-6 * g.norm())
+    if P == 1:
+        return
+
+    class Half:  # the other shards' (count, sum), centred squares and backward sums, added to this one's
+        def __init__(self, parts):
+            self.parts = list(parts)
+
+        def size(self):
+            return P
+
+        def all_reduce(self, t, op):
+            t += self.parts.pop(0).to(t.dtype)
+
+    xs, gs = [t.double() for t in x.chunk(P, 2)], [t.double() for t in g.chunk(P, 2)]
+    seg = [t.reshape(shape[0], G, -1) for t in xs]
+    n = sum(t.shape[-1] for t in seg)
+    mean = sum(t.sum(-1) for t in seg) / n
+    sq = [((t - mean[..., None]) ** 2).sum(-1) for t in seg]
+    rstd = (sum(sq) / n + 1e-5) ** -0.5
+    wd = torch.ones(shape[1], device=dev, dtype=torch.float64) if w is None else w.double()
+    gw_ = [(t * wd.reshape(1, -1, *[1] * (len(shape) - 2))).reshape(shape[0], G, -1) for t in gs]
+    xn = [(t - mean[..., None]) * rstd[..., None] for t in seg]
+    rest = lambda f: sum(f(i) for i in range(1, P))  # noqa: E731
+    others = Half([rest(lambda i: torch.stack([torch.full_like(mean, seg[i].shape[-1]), seg[i].sum(-1)], -1)), rest(lambda i: sq[i]),
+                   rest(lambda i: torch.stack([gw_[i].sum(-1), (gw_[i] * xn[i]).sum(-1)], -1))])
+    x0 = x.chunk(P, 2)[0].clone().requires_grad_()
+    y0 = jgn.group_norm(x0, G, w, b, (others,))
+    g0, = torch.autograd.grad(y0, x0, g.chunk(P, 2)[0])
+    assert not others.parts and rel_l2(y0, want.chunk(P, 2)[0]) < tol and rel_l2(g0, grads[0].chunk(P, 2)[0]) < tol
