@@ -212,6 +212,12 @@ int jg_roll_unpack_pack(void* x, const void* recv1, int axis1, int64_t window1, 
  * (local_mean / local_var of _functional.py:46-47). */
 int jg_ln_partial_fwd(float* mean, float* var, const void* x, int64_t rows,
                       int64_t cols, int x_dtype, void* stream);
+/* The same with a second copy of the means (NULL: none): the caller averages one over the group and still needs its
+ * own for jg_ln_recentre. */
+int jg_ln_partial_fwd2(float* mean, float* mean2, float* var, const void* x, int64_t rows, int64_t cols, int x_dtype,
+                       void* stream);
+/* var[r] += (local_mean[r] - mean[r])^2 (_functional.py:52): what is averaged over the group for the variance. */
+int jg_ln_recentre(float* var, const float* local_mean, const float* mean, int64_t rows, void* stream);
 
 /* x_hat = (x - mean) / sqrt(var + eps);  y = w * x_hat + b  (_functional.py:55-58)
  * with the COMBINED statistics. Also writes std[r] = sqrt(var[r] + eps), the
@@ -221,6 +227,11 @@ int jg_ln_apply(void* y, void* x_hat, float* std_out, const void* x,
                 const float* mean, const float* var, const void* w, const void* b,
                 int64_t rows, int64_t cols, float eps, int x_dtype, int out_dtype,
                 void* stream);
+/* The same with var_out[r] = var[r] + eps in out_dtype (NULL: none) and, when it is given, std_out the root of
+ * that rounded value, which is what _LayerNorm hands out and saves (_functional.py:57, 75). */
+int jg_ln_apply2(void* y, void* x_hat, float* std_out, void* var_out, const void* x, const float* mean, const float* var,
+                 const void* w, const void* b, int64_t rows, int64_t cols, float eps, int x_dtype, int out_dtype,
+                 void* stream);
 
 /* Backward partials (_functional.py:150-168), one pass over g and x_hat:
  *   mean_gxn[r] = mean_c(g*w), dot_gxn_xhat[r] = sum_c(g*w*x_hat)   (per row)
@@ -233,6 +244,11 @@ int jg_ln_partial_bwd(float* mean_gxn, float* dot_gxn_xhat, float* gw, float* gb
                       const void* g, const void* x_hat, const void* w, int64_t rows,
                       int64_t cols, int dtype, void* workspace, size_t workspace_bytes,
                       void* stream);
+
+/* The same with gw / gb in grad_dtype. */
+int jg_ln_partial_bwd2(float* mean_gxn, float* dot_gxn_xhat, void* gw, void* gb, int grad_dtype, const void* g,
+                       const void* x_hat, const void* w, int64_t rows, int64_t cols, int dtype, void* workspace,
+                       size_t workspace_bytes, void* stream);
 
 /* jg_ln_partial_bwd without a workspace argument, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, harnesses that

@@ -113,6 +113,18 @@ SIGNATURES: dict[str, tuple] = {
     ),
     "jg_roll_unpack": (c_int, [c_void_p, c_void_p, c_int, POINTER(c_int64), c_int, c_int64, c_int, c_void_p]),
     "jg_ln_partial_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int, c_void_p]),
+    "jg_ln_partial_fwd2": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int, c_void_p]),
+    "jg_ln_recentre": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
+    "jg_ln_apply2": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64,
+         c_float, c_int, c_int, c_void_p],
+    ),
+    "jg_ln_partial_bwd2": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int, c_void_p,
+         c_size_t, c_void_p],
+    ),
     "jg_ln_apply": (
         c_int,
         [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_float,

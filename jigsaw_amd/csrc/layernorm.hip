@@ -84,8 +84,8 @@ __device__ __forceinline__ void store_vec(typename Elem<DT>::T* row, long long c
 // ---------------------------------------------------------- partial statistics
 template <int DT>
 __global__ __launch_bounds__(kThreads) void ln_partial_fwd_kernel(
-    float* __restrict__ mean, float* __restrict__ var, const typename Elem<DT>::T* __restrict__ x,
-    long long rows, long long cols, bool vec_ok) {
+    float* __restrict__ mean, float* __restrict__ mean2, float* __restrict__ var,
+    const typename Elem<DT>::T* __restrict__ x, long long rows, long long cols, bool vec_ok) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const float inv = 1.0f / (float)cols;
@@ -113,16 +113,39 @@ __global__ __launch_bounds__(kThreads) void ln_partial_fwd_kernel(
     q = wave_sum(q) * inv;
     if (lane == 0) {
       mean[r] = m;
+      if (mean2 != nullptr) mean2[r] = m;
       var[r] = q;
     }
   }
 }
 
 // ----------------------------------------------------------------------- apply
+// std[r] = sqrt(var + eps); with var_out also v = var + eps in the output dtype and std = sqrt(v) of the rounded value, as
+// the reference keeps them for its backward (_functional.py:57, 75)
+template <int ODT>
+__device__ __forceinline__ void store_std(float* std_out, typename Elem<ODT>::T* var_out, long long r, float v) {
+  if (var_out != nullptr) {
+    const typename Elem<ODT>::T h = Elem<ODT>::down(v);
+    var_out[r] = h;
+    v = Elem<ODT>::up(h);
+  }
+  if (std_out != nullptr) std_out[r] = sqrtf(v);
+}
+
+// var[r] += (local_mean[r] - mean[r])^2: a shard's contribution to the variance about the common mean
+__global__ __launch_bounds__(kThreads) void ln_recentre_kernel(float* __restrict__ var, const float* __restrict__ local_mean,
+                                                               const float* __restrict__ mean, long long rows) {
+  const long long r = (long long)blockIdx.x * kThreads + threadIdx.x;
+  if (r >= rows) return;
+  const float d = local_mean[r] - mean[r];
+  var[r] = fmaf(d, d, var[r]);
+}
+
 template <int XDT, int ODT>
 __global__ __launch_bounds__(kThreads) void ln_apply_kernel(
     typename Elem<ODT>::T* __restrict__ y, typename Elem<ODT>::T* __restrict__ x_hat,
-    float* __restrict__ std_out, const typename Elem<XDT>::T* __restrict__ x,
+    float* __restrict__ std_out, typename Elem<ODT>::T* __restrict__ var_out,
+    const typename Elem<XDT>::T* __restrict__ x,
     const float* __restrict__ mean, const float* __restrict__ var,
     const typename Elem<ODT>::T* __restrict__ w, const typename Elem<ODT>::T* __restrict__ b,
     long long rows, long long cols, float eps, bool vx_ok, bool vo_ok, bool vw_ok) {
@@ -132,7 +155,7 @@ __global__ __launch_bounds__(kThreads) void ln_apply_kernel(
        r += (long long)gridDim.x * kWavesPerBlock) {
     const float m = mean[r];
     const float sd = sqrtf(var[r] + eps);
-    if (lane == 0 && std_out != nullptr) std_out[r] = sd;
+    if (lane == 0) store_std<ODT>(std_out, var_out, r, var[r] + eps);
     for (long long c = (long long)lane * kVec; c < cols; c += kWave * kVec) {
       float v[kVec], wv[kVec], bv[kVec], xh[kVec], out[kVec];
       load_vec<XDT>(x + r * cols, c, cols, vx_ok, v);
@@ -231,8 +254,12 @@ __global__ __launch_bounds__(kThreads) void ln_partial_bwd_kernel(
 // coalesced); its 16 wavefronts take the block partials k = w, w + 16, ... in 4 independent
 // chains each, and the 64 chain sums are added in a fixed order (deterministic).
 constexpr int kReduceWaves = 16;
-__global__ __launch_bounds__(kReduceWaves * 64) void ln_colreduce_kernel(float* __restrict__ gw,
-                                                                         float* __restrict__ gb,
+__device__ __forceinline__ void store_as(void* p, long long i, float v, int dtype) {
+  if (dtype == JG_F32) static_cast<float*>(p)[i] = v;
+  else if (dtype == JG_BF16) static_cast<uint16_t*>(p)[i] = Elem<JG_BF16>::down(v);
+  else static_cast<Elem<JG_F16>::T*>(p)[i] = Elem<JG_F16>::down(v);
+}
+__global__ __launch_bounds__(kReduceWaves * 64) void ln_colreduce_kernel(void* __restrict__ gw, void* __restrict__ gb, int dtype,
                                                                          const float* __restrict__ part,
                                                                          int nblocks, long long cols) {
   __shared__ float red[kReduceWaves][2][64];
@@ -263,8 +290,8 @@ __global__ __launch_bounds__(kReduceWaves * 64) void ln_colreduce_kernel(float* 
     sw += red[i][0][lane];
     sb += red[i][1][lane];
   }
-  if (gw != nullptr) gw[c] = sw;
-  if (gb != nullptr) gb[c] = sb;
+  if (gw != nullptr) store_as(gw, c, sw, dtype);
+  if (gb != nullptr) store_as(gb, c, sb, dtype);
 }
 
 template <int DT>
@@ -693,8 +720,8 @@ __device__ __forceinline__ void unpack8(const Raw8<DT>& in, bool ok, float out[k
 
 template <int DT, int CH, int U>
 __global__ __launch_bounds__(kThreads) void ln_partial_fwd_rows_kernel(
-    float* __restrict__ mean, float* __restrict__ var, const typename Elem<DT>::T* __restrict__ x,
-    long long rows, int cols, int G) {
+    float* __restrict__ mean, float* __restrict__ mean2, float* __restrict__ var,
+    const typename Elem<DT>::T* __restrict__ x, long long rows, int cols, int G) {
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int sl = lane & (G - 1), sub = lane / G, rpw = kWave / G;
   const float inv = 1.0f / (float)cols;
@@ -755,6 +782,7 @@ __global__ __launch_bounds__(kThreads) void ln_partial_fwd_rows_kernel(
       if (live[u] && sl == 0) {
         const long long r = r0 + u * stride + sub;
         mean[r] = m[u];
+        if (mean2 != nullptr) mean2[r] = m[u];
         var[r] = qs[u] * inv;
       }
     }
@@ -764,7 +792,8 @@ __global__ __launch_bounds__(kThreads) void ln_partial_fwd_rows_kernel(
 template <int XDT, int ODT, int CH, int U>
 __global__ __launch_bounds__(kThreads) void ln_apply_rows_kernel(
     typename Elem<ODT>::T* __restrict__ y, typename Elem<ODT>::T* __restrict__ x_hat,
-    float* __restrict__ std_out, const typename Elem<XDT>::T* __restrict__ x,
+    float* __restrict__ std_out, typename Elem<ODT>::T* __restrict__ var_out,
+    const typename Elem<XDT>::T* __restrict__ x,
     const float* __restrict__ mean, const float* __restrict__ var,
     const typename Elem<ODT>::T* __restrict__ w, const typename Elem<ODT>::T* __restrict__ b,
     long long rows, int cols, float eps, int G) {
@@ -796,7 +825,7 @@ __global__ __launch_bounds__(kThreads) void ln_apply_rows_kernel(
       if (!live[u]) continue;
       const long long r = r0 + u * stride + sub;
       const float s = sqrtf(sd[u] + eps);
-      if (sl == 0 && std_out != nullptr) std_out[r] = s;
+      if (sl == 0) store_std<ODT>(std_out, var_out, r, sd[u] + eps);
 #pragma unroll
       for (int k = 0; k < CH; ++k) {
         const int c = (k * G + sl) * kPlainVec;
@@ -1043,6 +1072,11 @@ void launch_plain_bwd(void* gx, float* part, const void* g, const void* x, const
 
 extern "C" int jg_ln_partial_fwd(float* mean, float* var, const void* x, int64_t rows,
                                  int64_t cols, int x_dtype, void* stream) {
+  return jg_ln_partial_fwd2(mean, nullptr, var, x, rows, cols, x_dtype, stream);
+}
+
+extern "C" int jg_ln_partial_fwd2(float* mean, float* mean2, float* var, const void* x, int64_t rows, int64_t cols,
+                                  int x_dtype, void* stream) {
   JG_REQUIRE(mean && var && x, "jg_ln_partial_fwd: NULL pointer");
   JG_REQUIRE(rows >= 0 && cols >= 1, "jg_ln_partial_fwd: bad shape (%lld, %lld)",
              (long long)rows, (long long)cols);
@@ -1056,11 +1090,11 @@ extern "C" int jg_ln_partial_fwd(float* mean, float* var, const void* x, int64_t
   if (in_regs)                                                                                     \
     with_row_shape<4>(cols, [&](auto ch, auto u) {                                                 \
       ln_partial_fwd_rows_kernel<DT, decltype(ch)::value, decltype(u)::value>                      \
-          <<<blocks, kThreads, 0, s>>>(mean, var, static_cast<const Elem<DT>::T*>(x), rows, (int)cols, G); \
+          <<<blocks, kThreads, 0, s>>>(mean, mean2, var, static_cast<const Elem<DT>::T*>(x), rows, (int)cols, G); \
     });                                                                                            \
   else                                                                                             \
     ln_partial_fwd_kernel<DT><<<row_grid(rows), kThreads, 0, s>>>(                                 \
-        mean, var, static_cast<const Elem<DT>::T*>(x), rows, cols, v)
+        mean, mean2, var, static_cast<const Elem<DT>::T*>(x), rows, cols, v)
   if (x_dtype == JG_F32) JG_GO(JG_F32);
   else if (x_dtype == JG_BF16) JG_GO(JG_BF16);
   else JG_GO(JG_F16);
@@ -1070,7 +1104,7 @@ extern "C" int jg_ln_partial_fwd(float* mean, float* var, const void* x, int64_t
 }
 
 template <int XDT, int ODT>
-static void launch_apply(void* y, void* x_hat, float* std_out, const void* x, const float* mean,
+static void launch_apply(void* y, void* x_hat, float* std_out, void* var_out, const void* x, const float* mean,
                          const float* var, const void* w, const void* b, int64_t rows,
                          int64_t cols, float eps, hipStream_t s) {
   typedef typename Elem<XDT>::T XT;
@@ -1082,26 +1116,42 @@ static void launch_apply(void* y, void* x_hat, float* std_out, const void* x, co
     const int G = plain_group(cols), blocks = plain_blocks(rows, cols, 2048);
     with_row_shape<2>(cols, [&](auto ch, auto u) {
       ln_apply_rows_kernel<XDT, ODT, decltype(ch)::value, decltype(u)::value><<<blocks, kThreads, 0, s>>>(
-          static_cast<OT*>(y), static_cast<OT*>(x_hat), std_out, static_cast<const XT*>(x), mean, var,
+          static_cast<OT*>(y), static_cast<OT*>(x_hat), std_out, static_cast<OT*>(var_out), static_cast<const XT*>(x), mean, var,
           static_cast<const OT*>(w), static_cast<const OT*>(b), rows, (int)cols, eps, G);
     });
     return;
   }
   ln_apply_kernel<XDT, ODT><<<row_grid(rows), kThreads, 0, s>>>(
-      static_cast<OT*>(y), static_cast<OT*>(x_hat), std_out, static_cast<const XT*>(x), mean, var,
+      static_cast<OT*>(y), static_cast<OT*>(x_hat), std_out, static_cast<OT*>(var_out), static_cast<const XT*>(x), mean, var,
       static_cast<const OT*>(w), static_cast<const OT*>(b), rows, cols, eps, vx, vo, vw);
+}
+
+extern "C" int jg_ln_recentre(float* var, const float* local_mean, const float* mean, int64_t rows, void* stream) {
+  JG_REQUIRE(var && local_mean && mean && rows >= 0, "jg_ln_recentre: bad argument");
+  if (rows == 0) return JG_OK;
+  JG_REQUIRE((rows + kThreads - 1) / kThreads < (1ll << 31), "jg_ln_recentre: too many rows");
+  ln_recentre_kernel<<<(unsigned)((rows + kThreads - 1) / kThreads), kThreads, 0, static_cast<hipStream_t>(stream)>>>(
+      var, local_mean, mean, rows);
+  JG_CHECK_LAUNCH("jg_ln_recentre");
+  return JG_OK;
 }
 
 extern "C" int jg_ln_apply(void* y, void* x_hat, float* std_out, const void* x,
                            const float* mean, const float* var, const void* w, const void* b,
                            int64_t rows, int64_t cols, float eps, int x_dtype, int out_dtype,
                            void* stream) {
+  return jg_ln_apply2(y, x_hat, std_out, nullptr, x, mean, var, w, b, rows, cols, eps, x_dtype, out_dtype, stream);
+}
+
+extern "C" int jg_ln_apply2(void* y, void* x_hat, float* std_out, void* var_out, const void* x, const float* mean,
+                            const float* var, const void* w, const void* b, int64_t rows, int64_t cols, float eps,
+                            int x_dtype, int out_dtype, void* stream) {
   JG_REQUIRE(y && x && mean && var && w, "jg_ln_apply: NULL pointer");
   JG_REQUIRE(rows >= 0 && cols >= 1, "jg_ln_apply: bad shape");
   JG_REQUIRE(known(x_dtype) && known(out_dtype), "jg_ln_apply: unknown dtype");
   if (rows == 0) return JG_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define JG_GO(X, O) launch_apply<X, O>(y, x_hat, std_out, x, mean, var, w, b, rows, cols, eps, s)
+#define JG_GO(X, O) launch_apply<X, O>(y, x_hat, std_out, var_out, x, mean, var, w, b, rows, cols, eps, s)
   if (x_dtype == out_dtype) {
     if (x_dtype == JG_F32) JG_GO(JG_F32, JG_F32);
     else if (x_dtype == JG_BF16) JG_GO(JG_BF16, JG_BF16);
@@ -1168,6 +1218,14 @@ extern "C" int jg_ln_partial_bwd(float* mean_gxn, float* dot_gxn_xhat, float* gw
                                  const void* g, const void* x_hat, const void* w, int64_t rows,
                                  int64_t cols, int dtype, void* workspace,
                                  size_t workspace_bytes, void* stream) {
+  return jg_ln_partial_bwd2(mean_gxn, dot_gxn_xhat, gw, gb, JG_F32, g, x_hat, w, rows, cols, dtype, workspace,
+                            workspace_bytes, stream);
+}
+
+extern "C" int jg_ln_partial_bwd2(float* mean_gxn, float* dot_gxn_xhat, void* gw, void* gb, int grad_dtype, const void* g,
+                                  const void* x_hat, const void* w, int64_t rows, int64_t cols, int dtype, void* workspace,
+                                  size_t workspace_bytes, void* stream) {
+  JG_REQUIRE(known(grad_dtype), "jg_ln_partial_bwd: unknown gradient dtype %d", grad_dtype);
   JG_REQUIRE(mean_gxn && dot_gxn_xhat && g && x_hat && w, "jg_ln_partial_bwd: NULL pointer");
   JG_REQUIRE(rows >= 0 && cols >= 1, "jg_ln_partial_bwd: bad shape");
   JG_REQUIRE(known(dtype), "jg_ln_partial_bwd: unknown dtype %d", dtype);
@@ -1191,7 +1249,7 @@ extern "C" int jg_ln_partial_bwd(float* mean_gxn, float* dot_gxn_xhat, float* gw
   if (rc) return rc;
   JG_CHECK_LAUNCH("jg_ln_partial_bwd");
   if (want_cols) {
-    ln_colreduce_kernel<<<jg::cdiv(cols, 64), kReduceWaves * 64, 0, s>>>(gw, gb, part, nparts, cols);
+    ln_colreduce_kernel<<<jg::cdiv(cols, 64), kReduceWaves * 64, 0, s>>>(gw, gb, grad_dtype, part, nparts, cols);
     JG_CHECK_LAUNCH("jg_ln_partial_bwd(colreduce)");
   }
   return JG_OK;
@@ -1351,7 +1409,7 @@ static int plain_bwd_common(const char* who, void* gx, float* gw, float* gb, con
   if (rows == 0) {
     // no rows: the column sums are zero (a fill kernel, so that the call can be captured in a graph)
     if (want_cols) {
-      ln_colreduce_kernel<<<(unsigned)((cols + 63) / 64), kReduceWaves * 64, 0, s>>>(gw, gb, nullptr, 0, cols);
+      ln_colreduce_kernel<<<(unsigned)((cols + 63) / 64), kReduceWaves * 64, 0, s>>>(gw, gb, JG_F32, nullptr, 0, cols);
       JG_CHECK_LAUNCH(who);
     }
     return JG_OK;
@@ -1377,7 +1435,7 @@ static int plain_bwd_common(const char* who, void* gx, float* gw, float* gb, con
 #undef JG_GO
   JG_CHECK_LAUNCH(who);
   if (want_cols) {
-    ln_colreduce_kernel<<<(unsigned)((cols + 63) / 64), kReduceWaves * 64, 0, s>>>(gw, gb, part, plain_blocks(rows, cols), cols);
+    ln_colreduce_kernel<<<(unsigned)((cols + 63) / 64), kReduceWaves * 64, 0, s>>>(gw, gb, JG_F32, part, plain_blocks(rows, cols), cols);
     JG_CHECK_LAUNCH(who);
   }
   return JG_OK;

@@ -76,23 +76,31 @@ class _LayerNorm(PositionalFunction):
         b = None if bias is None else bias.to(cdt).contiguous()
         cols = x.shape[-1]
         rows = x.numel() // cols
-        local_mean, local_var = partial_stats(x)
+        lib, dev, stream = _lib.load(), x.device, _lib.stream_ptr(x.device)
+        stat_shape = x.shape[:-1] + (1,)
+        sharded = _group_size(channel_group) > 1
+        # the mean that is averaged over the group, the variance, the rank's own mean, and the root the backward wants
+        mean, var, local_mean, std = torch.empty((4, *stat_shape), dtype=torch.float32, device=dev).unbind(0)
+        rc = lib.jg_ln_partial_fwd2(_lib.ptr(mean), _lib.ptr(local_mean if sharded else None), _lib.ptr(var), _lib.ptr(x),
+                                    rows, cols, _lib.dtype_code(x.dtype), stream)
+        _lib.check(rc, "jg_ln_partial_fwd2")
+        if sharded:
+            _all_reduce(mean, "avg", channel_group)
+            rc = lib.jg_ln_recentre(_lib.ptr(var), _lib.ptr(local_mean), _lib.ptr(mean), rows, stream)
+            _lib.check(rc, "jg_ln_recentre")
+            _all_reduce(var, "avg", channel_group)
 
-        mean = local_mean.clone()
-        _all_reduce(mean, "avg", channel_group)
-        var = local_var + (local_mean - mean) ** 2 if _group_size(channel_group) > 1 else local_var
-        _all_reduce(var, "avg", channel_group)
-
-        y = torch.empty(x.shape, dtype=cdt, device=x.device)
+        y = torch.empty(x.shape, dtype=cdt, device=dev)
         x_norm = torch.empty_like(y)
-        rc = _lib.load().jg_ln_apply(
-            _lib.ptr(y), _lib.ptr(x_norm), None, _lib.ptr(x), _lib.ptr(mean), _lib.ptr(var),
-            _lib.ptr(w), _lib.ptr(b), rows, cols, float(eps),
-            _lib.dtype_code(x.dtype), _lib.dtype_code(cdt), _lib.stream_ptr(x.device),
+        var_eps = torch.empty(stat_shape, dtype=cdt, device=dev)
+        rc = lib.jg_ln_apply2(
+            _lib.ptr(y), _lib.ptr(x_norm), _lib.ptr(std), _lib.ptr(var_eps), _lib.ptr(x), _lib.ptr(mean), _lib.ptr(var),
+            _lib.ptr(w), _lib.ptr(b), rows, cols, float(eps), _lib.dtype_code(x.dtype), _lib.dtype_code(cdt), stream,
         )
-        _lib.check(rc, "jg_ln_apply")
+        _lib.check(rc, "jg_ln_apply2")
+        var_eps._jg_std = std  # read by setup_context: the root of var_eps, formed on the way
         # an input returned as-is cannot be saved by setup_context: hand out a view
-        return y, x_norm, (w.view_as(w) if w is weight else w), (var + eps).to(cdt)
+        return y, x_norm, (w.view_as(w) if w is weight else w), var_eps
 
     @staticmethod
     def setup_context(ctx, inputs, output):  # noqa: D102
@@ -105,7 +113,8 @@ class _LayerNorm(PositionalFunction):
         ctx.param_dtypes = (weight.dtype, None if bias is None else bias.dtype)
         ctx.in_dtype = x.dtype
         # sqrt(var + eps), as the reference saves it (_functional.py:75); fp32 for the kernels
-        ctx.save_for_backward(x_norm, w, torch.sqrt(var.to(torch.float32)))
+        std = getattr(var, "_jg_std", None)
+        ctx.save_for_backward(x_norm, w, torch.sqrt(var.to(torch.float32)) if std is None else std)
 
     @staticmethod
     def backward(ctx, grad_output, x_norm_grad, weight_grad, var_grad):  # noqa: D102
@@ -120,19 +129,21 @@ class _LayerNorm(PositionalFunction):
         lib = _lib.load()
         dev = g.device
 
-        mean_gxn = torch.empty_like(std)
-        dot = torch.empty_like(std)
+        mean_gxn, dot = torch.empty((2, *std.shape), dtype=torch.float32, device=dev).unbind(0)
         need_w = ctx.needs_input_grad[1]
         need_b = ctx.has_bias and ctx.needs_input_grad[2]
-        gw = torch.empty(cols, dtype=torch.float32, device=dev) if need_w else None
-        gb = torch.empty(cols, dtype=torch.float32, device=dev) if need_b else None
+        # the column sums leave the kernel in the parameters' dtype where they share one
+        wdt, bdt = ctx.param_dtypes
+        gdt = wdt if wdt in _lib._DTYPES and bdt in (None, wdt) else torch.float32
+        gw = torch.empty(cols, dtype=gdt, device=dev) if need_w else None
+        gb = torch.empty(cols, dtype=gdt, device=dev) if need_b else None
         ws_bytes = int(lib.jg_ln_bwd_workspace_bytes(rows, cols)) if (need_w or need_b) else 0
         ws = torch.empty(max(ws_bytes, 4), dtype=torch.uint8, device=dev)
-        rc = lib.jg_ln_partial_bwd(
-            _lib.ptr(mean_gxn), _lib.ptr(dot), _lib.ptr(gw), _lib.ptr(gb), _lib.ptr(g), _lib.ptr(x_norm),
+        rc = lib.jg_ln_partial_bwd2(
+            _lib.ptr(mean_gxn), _lib.ptr(dot), _lib.ptr(gw), _lib.ptr(gb), _lib.dtype_code(gdt), _lib.ptr(g), _lib.ptr(x_norm),
             _lib.ptr(w), rows, cols, _lib.dtype_code(g.dtype), _lib.ptr(ws), ws_bytes, _lib.stream_ptr(dev),
         )
-        _lib.check(rc, "jg_ln_partial_bwd")
+        _lib.check(rc, "jg_ln_partial_bwd2")
 
         grad_x = None
         if ctx.needs_input_grad[0]:
@@ -145,7 +156,6 @@ class _LayerNorm(PositionalFunction):
             )
             _lib.check(rc, "jg_ln_bwd_apply")
             grad_x = grad_x.to(ctx.in_dtype)
-        wdt, bdt = ctx.param_dtypes
         grad_w = gw.to(wdt) if need_w else None
         grad_b = gb.to(bdt) if need_b else None
         return grad_x, grad_w, grad_b, None, None
