@@ -76,6 +76,8 @@ constexpr int CK = 16;                         // contraction channels per stage
 constexpr int STAGE_SLOTS = 2 * IN_ROWS * ROW_SLOTS;  // [kg][row][slot]
 constexpr int STAGE_BYTES = STAGE_SLOTS * 16;         // 41472
 constexpr int TASKS = 2 * IN_ROWS * OCTS;             // 324 tasks of 8 channels x 8 pixels
+constexpr int LANES_ODD = 64 / OCTS * OCTS;           // lanes of a wavefront with a task where rows start anywhere
+static_assert(2 * IN_ROWS <= WAVES * (LANES_ODD / OCTS), "every row of tasks has a wavefront");
 
 __device__ __forceinline__ int in_slot(int col) { return (col & 7) * OCTS + (col >> 3); }
 
@@ -256,9 +258,13 @@ __global__ __launch_bounds__(256) void prep_weights_split_kernel(uint16_t* __res
 }
 
 // ------------------------------------------------------------ forward kernel
-// EVEN: Win, pad_w and the plane size are even and x is 4-byte aligned, so every
-// pixel pair of a task is one aligned dword that is either wholly inside or wholly
-// outside the tensor. Otherwise the prefetch falls back to 2-byte loads.
+// EVEN: Win is even and x is 4-byte aligned, so that the 16 bytes of a task start on a dword. Otherwise
+// rows and channel planes start on odd pixels as often as not. 2-byte loads (64 of them per task) took
+// 68 us for 2 x 40 -> 72 channels of 217 x 301, where the kernel had to wait for nothing else; vector
+// loads at 2-byte aligned addresses run at a fraction of the rate. Such a task reads the 16 bytes from the
+// dword below its first pixel, and on their way to LDS the values move up by the odd pixel; the dword that
+// comes in at the end is the first one of the next task of the row, in the next lane (a wavefront therefore
+// holds 7 whole rows of 9 tasks).
 // 2-byte stores with a scalar base and a 32-bit lane offset. The epilogue issues 128 of
 // them per lane and tile; with the 64-bit lane addresses the compiler builds for plain
 // pointer code each one moves 512 bytes of addresses to the memory pipeline, which is what
@@ -346,9 +352,9 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   const size_t plane = (size_t)p.Hin * p.Win;
   const size_t chan_stride = plane * p.Din;            // elements between channels
   const uint32_t chan_b = (uint32_t)(chan_stride * 2);  // bytes
-  const bool has_task = tid < TASKS;
-  const int oct = tid % OCTS;
-  const int rr = tid / OCTS;         // = g8 * IN_ROWS + row
+  const bool has_task = EVEN ? tid < TASKS : lane < LANES_ODD && wave * (LANES_ODD / OCTS) + lane / OCTS < 2 * IN_ROWS;
+  const int oct = EVEN ? tid % OCTS : lane % OCTS;
+  const int rr = EVEN ? tid / OCTS : wave * (LANES_ODD / OCTS) + lane / OCTS;  // = g8 * IN_ROWS + row
   const int t_row = rr % IN_ROWS;
   const int t_col = oct * 8;
   const int g8 = rr / IN_ROWS;
@@ -359,6 +365,9 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   const uint32_t chan_bt = (uint32_t)(chan_stride_t * 2);
   const uint32_t t_off_t = (uint32_t)(((size_t)g8 * 8 * chan_stride_t + (size_t)t_row * p.tn_w + t_col) * 2);
   uint32_t stg[8][4];
+  bool stg_masked = false;    // wave-uniform: the staged window sticks out of the tensor
+  uint32_t stg_mask = 0xffu;  // this task's pixels inside the tensor (one bit each), where stg_masked
+  uint32_t stg_odd = 0;       // not EVEN: one bit per channel, the task starts on the upper half of a dword
 
   struct TileCoord {
     int n, od, th, tw;
@@ -448,6 +457,8 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
       const int dt = id - p.tlo_d;
       const char* origin_t = cur.base_t + 2 * ((ptrdiff_t)((size_t)cx0 * chan_stride_t) + (ptrdiff_t)dt * (ptrdiff_t)plane_t);
       if (dt >= 0 && dt < p.tn_d && cur.window_in_t) {
+        stg_masked = false;
+        stg_odd = 0;
         if (!has_task) return;
         // 4-byte aligned accesses only (2-byte aligned vector loads run at a fraction of the
         // rate): a window that starts on an odd column is read one pixel early and shifted.
@@ -494,54 +505,64 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
         return;
       }
     }
+    stg_masked = !interior;
     if (!has_task) return;
     const char* a = origin + t_off;
-    if (EVEN && interior) {
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const u32x4_a4 v = *reinterpret_cast<const u32x4_a4*>(a + (size_t)c * chan_b);
-        stg[c][0] = v.x; stg[c][1] = v.y; stg[c][2] = v.z; stg[c][3] = v.w;
-      }
-    } else if (EVEN) {
-      // A window that sticks out of the tensor (the border tiles of a padded problem: one tile in
-      // seven of configuration 2's input gradient). Most of its tasks still lie wholly inside and
-      // keep their 16-byte loads, the ones wholly outside load nothing; only the tasks that
-      // straddle an edge go dword by dword.
-      const int ih = ih0 + t_row, iw = iw0 + t_col;
-      const bool row_ok = depth_ok && (ih >= 0) && (ih < p.Hin);
-      if (row_ok && iw >= 0 && iw + 8 <= p.Win && cvalid >= 8) {
+    if (interior) {
+      if (EVEN) {
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
           const u32x4_a4 v = *reinterpret_cast<const u32x4_a4*>(a + (size_t)c * chan_b);
           stg[c][0] = v.x; stg[c][1] = v.y; stg[c][2] = v.z; stg[c][3] = v.w;
         }
-      } else if (!row_ok || iw + 8 <= 0 || iw >= p.Win) {
+      } else {
+        const char* down = reinterpret_cast<const char*>(reinterpret_cast<uintptr_t>(origin) & ~(uintptr_t)3);  // uniform
+        uint32_t off = t_off + (uint32_t)(reinterpret_cast<uintptr_t>(origin) & 3);
+        stg_odd = 0;
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
-          stg[c][0] = 0u; stg[c][1] = 0u; stg[c][2] = 0u; stg[c][3] = 0u;
+          const u32x4_a4 v = *reinterpret_cast<const u32x4_a4*>(down + (off & ~3u));
+          stg[c][0] = v.x; stg[c][1] = v.y; stg[c][2] = v.z; stg[c][3] = v.w;
+          stg_odd |= ((off >> 1) & 1u) << c;
+          off += chan_b;
         }
-      } else {
-        bool ok[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) ok[j] = iw + 2 * j >= 0 && iw + 2 * j + 2 <= p.Win;
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            stg[c][j] = (ok[j] && c < cvalid) ? *reinterpret_cast<const uint32_t*>(a + (size_t)c * chan_b + 4 * j) : 0u;
       }
     } else {
+      // A window that sticks out of the tensor, or whose 16 channels do (a ragged last step). A task reads
+      // its 16 bytes wherever they lie inside the tensor, also past the end of its row; store_stage clears
+      // the pixels that are not the row's. Tasks without any pixel of the tensor read the prepared weights
+      // instead, so that no load stands under a condition. What is left are the tasks whose bytes reach
+      // over the tensor's own ends: those go dword by dword.
       const int ih = ih0 + t_row, iw = iw0 + t_col;
-      const bool rows_ok = depth_ok && (ih >= 0) && (ih < p.Hin);
+      const bool row_ok = depth_ok && ih >= 0 && ih < p.Hin && cvalid > 0;
+      const int first = max(0, min(8, -iw)), past = max(0, min(8, p.Win - iw));
+      stg_mask = row_ok ? ((1u << past) - 1u) & ~((1u << first) - 1u) : 0u;
+      // (not EVEN: the task before takes its last pixel from this one's first dword)
+      const bool need = EVEN ? stg_mask != 0u : row_ok && iw - 1 < p.Win && iw + 8 > 0;
+      const uint32_t span = (uint32_t)(min(cvalid, 8) - 1) * chan_b;
+      const bool fits = a >= reinterpret_cast<const char*>(p.x) && a + (size_t)span + 16 <= p.x_end;
+      const char* from = need && fits ? a : reinterpret_cast<const char*>(p.wprep);
+      const uint32_t step = need && fits ? chan_b : 0u;
+      uint32_t off = 0;
+      stg_odd = 0;
 #pragma unroll
       for (int c = 0; c < 8; ++c) {
-        const bool row_ok = rows_ok && c < cvalid;
-        const uint16_t* e = reinterpret_cast<const uint16_t*>(a + (size_t)c * chan_b);
+        const uintptr_t at = reinterpret_cast<uintptr_t>(from) + off;
+        const u32x4_a4 v = *reinterpret_cast<const u32x4_a4*>(EVEN ? at : at & ~(uintptr_t)3);
+        stg[c][0] = v.x; stg[c][1] = v.y; stg[c][2] = v.z; stg[c][3] = v.w;
+        if (!EVEN) stg_odd |= (uint32_t)((at >> 1) & 1) << c;
+        off += c + 1 < cvalid ? step : 0u;
+      }
+      if (__builtin_amdgcn_ballot_w64(need && !fits) != 0 && need && !fits) {
+        stg_odd = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t lo = (row_ok && iw + 2 * j >= 0 && iw + 2 * j < p.Win) ? (uint32_t)e[2 * j] : 0u;
-          const uint32_t hi = (row_ok && iw + 2 * j + 1 >= 0 && iw + 2 * j + 1 < p.Win) ? (uint32_t)e[2 * j + 1] : 0u;
-          stg[c][j] = lo | (hi << 16);
+        for (int c = 0; c < 8; ++c) {
+          const uintptr_t at = reinterpret_cast<uintptr_t>(a) + (uint32_t)min(c, cvalid - 1) * (size_t)chan_b;
+          const char* d = reinterpret_cast<const char*>(at & ~(uintptr_t)3);
+          stg_odd |= (uint32_t)((at >> 1) & 1) << c;
+#pragma unroll
+          for (int j = 0; j < 4; ++j)  // a dword that holds a pixel of the tensor
+            stg[c][j] = d + 4 * j + 3 >= reinterpret_cast<const char*>(p.x) && d + 4 * j < p.x_end ? *reinterpret_cast<const uint32_t*>(d + 4 * j) : 0u;
         }
       }
     }
@@ -556,6 +577,26 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
         if (c >= cvalid) {
           stg[c][0] = 0u; stg[c][1] = 0u; stg[c][2] = 0u; stg[c][3] = 0u;
         }
+    }
+    if (!EVEN) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const uint32_t shift = ((stg_odd >> c) & 1u) << 4;
+        // the first dword of the next lane (wavefront shift left by one)
+        const uint32_t next = __builtin_amdgcn_update_dpp(0, stg[c][0], 0x130, 0xf, 0xf, false);
+        stg[c][0] = __builtin_amdgcn_alignbit(stg[c][1], stg[c][0], shift);
+        stg[c][1] = __builtin_amdgcn_alignbit(stg[c][2], stg[c][1], shift);
+        stg[c][2] = __builtin_amdgcn_alignbit(stg[c][3], stg[c][2], shift);
+        stg[c][3] = __builtin_amdgcn_alignbit(next, stg[c][3], shift);
+      }
+    }
+    if (stg_masked) {  // uniform
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t keep = (((stg_mask >> (2 * j)) & 1u) * 0xffffu) | (((stg_mask >> (2 * j + 1)) & 1u) * 0xffff0000u);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) stg[c][j] &= keep;
+      }
     }
     u32x4* row_base = lds_in + buf * STAGE_SLOTS + t_lds;
 #pragma unroll
@@ -1201,7 +1242,9 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
     const int org = L.pad_w % TW - TW;
     if ((L.Wout - org + TW - 1) / TW <= (L.Wout + TW - 1) / TW) p.org_w = org;
   }
-  p.lead = (L.pad_w - p.org_w) & 1;
+  // rows of the staged windows start at even columns where `lead` can see to it: 4-byte aligned loads
+  const bool even = (L.Win % 2 == 0) && ((reinterpret_cast<uintptr_t>(x16) & 3) == 0);
+  p.lead = even ? (L.pad_w - p.org_w) & 1 : 0;
   p.tiles_w = (L.Wout - p.org_w + TW - 1) / TW;
   p.sw = p.tiles_w;
   const long long tiles = (long long)L.N * L.Dout * p.tiles_h * p.tiles_w;
@@ -1224,8 +1267,6 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
   if (wgs > tiles) wgs = (int)tiles;
   wgs = (wgs + 7) & ~7;  // whole XCD rounds
   dim3 grid((unsigned)wgs, (unsigned)lay.mtiles, 1);
-  // rows of the staged windows start at even columns (`lead` sees to that): 4-byte aligned loads
-  const bool even = (L.Win % 2 == 0) && ((reinterpret_cast<uintptr_t>(x16) & 3) == 0);
   void (*kern)(StripTable, FwdParams) = nullptr;
   if (L.f16 && (L.fold || L.xt != nullptr))
     JG_FAIL(JG_ERR_UNSUPPORTED, "%s: the fold epilogue and the framed input are built for bf16 only", who);
