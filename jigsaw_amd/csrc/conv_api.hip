@@ -202,7 +202,8 @@ extern "C" int jg_conv_wgrad_bias(void* gw, void* gb, const void* x, const void*
   if (rc) return rc;
   JG_REQUIRE(gw && gb && x && go, "jg_conv_wgrad_bias: NULL pointer");
   JG_REQUIRE(known(dtype), "jg_conv_wgrad_bias: unknown dtype %d", dtype);
-  if (dtype != JG_BF16 || !jg::mfma_wgrad_supported(g, dtype))
-    JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_wgrad_bias: geometry / dtype only has the separate kernels");
-  return jg::mfma_wgrad(gw, gb, x, go, g, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+  if (!jg::mfma_wgrad_supported(g, dtype))
+    JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_wgrad_bias: geometry only has the separate kernels");
+  return jg::mfma_wgrad(gw, gb, x, go, g, workspace, workspace_bytes, static_cast<hipStream_t>(stream), nullptr, nullptr, nullptr,
+                        dtype);
 }

@@ -1,6 +1,6 @@
 // Weight gradient of the 3x3 (2-D) and 3x3x3 (3-D) convolution on the bf16 matrix
-// cores, stride 1, dilation 1, channels-first tensors; a launch covers a block of 32 or
-// 64 channels a side, any other channel counts are walked block by block. Optionally the
+// cores, stride 1, dilation 1, channels-first tensors; a workgroup covers a block of 32 or
+// 64 channels a side, any other channel counts are more blocks of the same launch. Optionally the
 // bias gradient from the same pass over g. fp16 tensors run the same kernel on the fp16
 // MFMA instruction (the gradient is reduced in fp32 and rounded to fp16 once); fp32 tensors
 // run as sums of three bf16 parts per operand ("split mode": the parts are extra channels,
@@ -35,9 +35,11 @@
 //               channel-lanes of a fragment read hit distinct banks.
 //   Bias grad   the lanes that carry the g chunks to LDS add them up on the way
 //               (fp32), one partial per workgroup and channel.
-//   Reduction   every wavefront writes its partial to the workspace; a second kernel
-//               sums the partials in a fixed order (deterministic) and writes gw in
-//               the weight layout.
+//   Reduction   the two column halves of a pair are added in LDS, the workgroup's partial goes
+//               to the workspace; a second kernel sums the partials in a fixed order
+//               (deterministic) and writes gw in the weight layout and gb, in their own dtype.
+#include <cmath>
+
 #include "conv_common.h"
 
 namespace {
@@ -47,6 +49,7 @@ using jg::mfma_frame_bands;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -63,21 +66,24 @@ struct WgradParams {
   const uint16_t* x;  // (N, Cin, Din, Hin, Win)
   const uint16_t* g;  // (N, Cout, Dout, Hout, Wout)
   const char* x_end;  // one past the last byte of x
-  float* part;        // [wavefront slot][tap9][co][c']
-  float* bias_part;   // [workgroup][co] or NULL
+  const char* g_end;  // one past the last byte of g
+  float* part;        // [block][workgroup][tap9][32 x 32 pair][4][lane][4] (see the end of the kernel)
+  float* bias_part;   // [block][workgroup][co], written by the blocks at the first x channel, or NULL
   // Framed input: xt (N, Cin, tn_d, tn_h, tn_w) is the own tile, at [tlo, tlo + tn) inside x.
   // A row pair whose window lies inside the tile is read from xt. NULL: all from x.
   const uint16_t* xt;
   int tlo_d, tlo_h, tlo_w, tn_d, tn_h, tn_w;
-  int Cin, Cout;            // channels of the block this launch works on (32 or 64 a side)
-  int cin_valid, cout_valid;  // how many of them exist; the others repeat the last one and are dropped
-  int cin_total, cout_total;  // channels of the tensors (batch strides); x and g point at the block's first
+  // Blocks of channels, one per blockIdx.y: (block of g channels, block of x channels, part pair), the pair
+  // fastest. cin, cout are the channels of one part (plain tensors have one), pair k multiplies part
+  // (gparts >> 2 k) & 3 of g with part (xparts >> 2 k) & 3 of x. A channel past the last one repeats it and
+  // is dropped where the partial sums are added up.
+  int cin, cout, ci_blocks, npairs;
+  uint32_t gparts, xparts;
+  int cin_total, cout_total;  // channels of the tensors (parts * cin, parts * cout): batch strides
   int Din, Hin, Win, Dout, Hout, Wout;
   int pad_d, pad_h, pad_w;
   int row_pairs, col_tiles;
   long long total_stages;  // N * Dout * col_tiles * row_pairs
-  int w_first, w_last;     // what a stage of the first / last column strip costs, in stages of the other strips
-  int wd_first, wd_last;   // the same for every stage of the first / last output depth (1: a plane like the others)
 };
 
 // Wavefronts per workgroup: (g block, x block) pairs x 2 column halves; a 6-wavefront
@@ -87,8 +93,17 @@ constexpr int wgrad_threads(int cgb, int cxb) {
   return (cgb * cxb * HALVES > 4) ? 512 : 64 * cgb * cxb * HALVES;
 }
 
-// sum of the 8 bf16 values of a chunk
-__device__ __forceinline__ float sum_bf16x8(const u32x4& v) {
+// sum of the 8 values of a chunk
+template <bool F16>
+__device__ __forceinline__ float sum_of_8(const u32x4& v) {
+  if (F16) {
+    const f16x8 h = __builtin_bit_cast(f16x8, v);
+    float s = (float)h[0] + (float)h[1];
+    s += (float)h[2] + (float)h[3];
+    s += (float)h[4] + (float)h[5];
+    s += (float)h[6] + (float)h[7];
+    return s;
+  }
   float s = __uint_as_float(v.x << 16) + __uint_as_float(v.x & 0xffff0000u);
   s += __uint_as_float(v.y << 16) + __uint_as_float(v.y & 0xffff0000u);
   s += __uint_as_float(v.z << 16) + __uint_as_float(v.z & 0xffff0000u);
@@ -97,7 +112,9 @@ __device__ __forceinline__ float sum_bf16x8(const u32x4& v) {
 }
 
 // F16: x and g hold fp16 instead of bf16 (v_mfma_f32_32x32x16_f16); the partial sums are fp32 either way.
-// EVEN: 0 = no assumption about the rows (every load checks its bounds), 1 = even row lengths,
+// EVEN: 0 = rows may start on odd pixels: a chunk is read from the dword below it, with the dword of its last
+// pixel, and moved into place on its way to LDS (2-byte loads took 52 us where this takes 23: 40 x 72
+// channels, 2 x 217 x 301), 1 = even row lengths,
 // 4-byte aligned tensors and an even padding across W, so that a stage's windows start on dwords and
 // the 16-byte vector loads apply, 2 = the same with an odd padding: the x window is staged from one
 // pixel earlier, where it is dword aligned again, and the fragments are built one pixel further in.
@@ -131,50 +148,27 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
   // Workgroups are dealt to the 8 XCDs round robin; the ranges are numbered so that one
   // XCD holds neighbouring column strips, whose x rows share cache lines in that XCD's L2.
   const unsigned wg_rank = gridDim.x % 8 == 0 ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
-  // The ranges hold equal cost, not equal counts: the stages of a column strip whose windows
-  // stick out of the tensor (or whose last columns do not exist) load with bounds checks and
-  // take several times as long, and a workgroup whose whole range lay in such a strip would set
-  // the kernel's time. Cost runs like the stages: per plane the first strip at w_first a
-  // stage, the middle strips at 1, the last at w_last; a plane at the first / last output depth
-  // whose depth taps stick out is slow as a whole (wd_first / wd_last a stage). With all four at
-  // 1 the ranges are counts.
-  const long long strip_first = (long long)p.row_pairs * p.w_first;
-  const long long strip_mid = (long long)p.row_pairs * (p.col_tiles > 2 ? p.col_tiles - 2 : 0);
-  const long long strip_last = p.col_tiles > 1 ? (long long)p.row_pairs * p.w_last : 0;
-  const long long plane_cost = strip_first + strip_mid + strip_last;
-  const long long plane_stages = (long long)p.row_pairs * p.col_tiles;
-  const long long head_cost = p.wd_first > 1 ? plane_stages * p.wd_first : plane_cost;
-  const long long tail_cost = p.Dout > 1 ? (p.wd_last > 1 ? plane_stages * p.wd_last : plane_cost) : 0;
-  const long long mid_cost = (p.Dout > 2 ? p.Dout - 2 : 0) * plane_cost;
-  const long long entry_cost = head_cost + mid_cost + tail_cost;  // one batch entry
-  const long long total_cost = (p.total_stages / (plane_stages * p.Dout)) * entry_cost;
-  auto in_plane = [&](long long rem) -> long long {  // stage inside a plane of ordinary cost
-    if (rem < strip_first) return rem / p.w_first;
-    if (rem < strip_first + strip_mid) return p.row_pairs + (rem - strip_first);
-    return (long long)p.row_pairs * (p.col_tiles - 1) + (rem - strip_first - strip_mid) / p.w_last;
-  };
-  auto stage_at = [&](long long cost) -> long long {
-    if (cost >= total_cost) return p.total_stages;
-    const long long n = cost / entry_cost;
-    long long rem = cost - n * entry_cost, od, st;
-    if (rem < head_cost) {
-      od = 0;
-      st = p.wd_first > 1 ? rem / p.wd_first : in_plane(rem);
-    } else if (rem < head_cost + mid_cost) {
-      rem -= head_cost;
-      const long long k = rem / plane_cost;
-      od = 1 + k;
-      st = in_plane(rem - k * plane_cost);
-    } else {
-      rem -= head_cost + mid_cost;
-      od = p.Dout - 1;
-      st = p.wd_last > 1 ? rem / p.wd_last : in_plane(rem);
-    }
-    return (n * p.Dout + od) * plane_stages + st;
-  };
-  const long long per = (total_cost + gridDim.x - 1) / gridDim.x;
-  const long long s_begin = stage_at(per * wg_rank);
-  const long long s_end = stage_at(per * (wg_rank + 1));
+  const long long per = (p.total_stages + gridDim.x - 1) / gridDim.x;
+  const long long s_begin = min(per * wg_rank, p.total_stages);
+  const long long s_end = min(per * (wg_rank + 1), p.total_stages);
+
+  // ---- the block of channels
+  constexpr int KD = CXB == 3 ? 3 : 1, CIN_B = XC / KD;  // three x blocks are the depth taps of 32 channels
+  int cin_valid, cout_valid;                             // channels of the block that exist
+  const uint16_t *xb, *gb;                               // its first channel in batch entry 0
+  const int block = blockIdx.y;
+  bool first_x;
+  {
+    const int pair_k = block % p.npairs, rest = block / p.npairs;
+    const int ci0 = (rest % p.ci_blocks) * CIN_B, co0 = (rest / p.ci_blocks) * GC;
+    const int gpart = (int)((p.gparts >> (2 * pair_k)) & 3u), xpart = (int)((p.xparts >> (2 * pair_k)) & 3u);
+    cin_valid = min(CIN_B, p.cin - ci0);
+    cout_valid = min(GC, p.cout - co0);
+    xb = p.x + (size_t)(xpart * p.cin + ci0) * ((size_t)p.Hin * p.Win * p.Din);
+    gb = p.g + (size_t)(gpart * p.cout + co0) * ((size_t)p.Hout * p.Wout * p.Dout);
+    first_x = ci0 == 0 && xpart == 0;  // the bias sum of these g rows is this block's
+  }
+  float* const bias_part = p.bias_part != nullptr && first_x ? p.bias_part : nullptr;
 
   const size_t plane_x = (size_t)p.Hin * p.Win, plane_g = (size_t)p.Hout * p.Wout;
   const size_t x_cs = plane_x * p.Din, g_cs = plane_g * p.Dout;  // channel strides
@@ -189,16 +183,16 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     const int q = tid + rd * THREADS;
     if (q < G_CHUNKS) {
       const int c8 = q & 7, r = (q >> 3) % SR, ch = q / (8 * SR);
-      const int che = ch < p.cout_valid ? ch : p.cout_valid - 1;  // a channel past the last one reads the last
+      const int che = ch < cout_valid ? ch : cout_valid - 1;  // a channel past the last one reads the last
       c_goff[rd] = (uint32_t)((che * g_cs + (size_t)r * p.Wout + c8 * 8) * 2);
       c_lds[rd] = (uint32_t)(ch * G_CH + r * (SW * 2) + c8 * 16);
     } else if (q < CHUNKS) {
       const int qx = q - G_CHUNKS;
       const int c8 = qx % X_CPR;
       const int rr = qx / X_CPR;
-      const int r2 = rr & 1, ch = rr >> 1;      // ch = kd * Cin + ci
-      const int kd = ch / p.Cin, cib = ch - kd * p.Cin;
-      const int ci = cib < p.cin_valid ? cib : p.cin_valid - 1;
+      const int r2 = rr & 1, ch = rr >> 1;      // ch = kd * CIN_B + ci
+      const int kd = ch / CIN_B, cib = ch - kd * CIN_B;
+      const int ci = cib < cin_valid ? cib : cin_valid - 1;
       c_goff[rd] = (uint32_t)((ci * x_cs + kd * plane_x + (size_t)r2 * p.Win + c8 * 8) * 2);
       c_lds[rd] = (uint32_t)(ch * X_CH + c8 * 16);
       x_second |= (uint32_t)r2 << rd;
@@ -213,8 +207,8 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
   uint32_t t_goff = 0, t_lds = 0;
   if (has_tail) {
     const int r2 = tid & 1, ch = tid >> 1;
-    const int kd = ch / p.Cin, cib = ch - kd * p.Cin;
-    const int ci = cib < p.cin_valid ? cib : p.cin_valid - 1;
+    const int kd = ch / CIN_B, cib = ch - kd * CIN_B;
+    const int ci = cib < cin_valid ? cib : cin_valid - 1;
     t_goff = (uint32_t)((ci * x_cs + kd * plane_x + (size_t)r2 * p.Win + SW) * 2);
     t_lds = (uint32_t)(ch * X_CH + SW * 2);
   }
@@ -232,14 +226,14 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
         const int qx = q - G_CHUNKS;
         const int c8 = qx % X_CPR, rr = qx / X_CPR;
         const int r2 = rr & 1, ch = rr >> 1;
-        const int kd = ch / p.Cin, ci = ch - kd * p.Cin;
+        const int kd = ch / CIN_B, ci = ch - kd * CIN_B;
         c_toff[rd] = (uint32_t)((ci * t_cs + kd * plane_t + (size_t)r2 * p.tn_w + c8 * 8) * 2);
         x_kd |= (uint32_t)kd << (2 * rd);
       }
     }
     if (has_tail) {
       const int r2 = tid & 1, ch = tid >> 1;
-      const int kd = ch / p.Cin, ci = ch - kd * p.Cin;
+      const int kd = ch / CIN_B, ci = ch - kd * CIN_B;
       t_toff = (uint32_t)((ci * t_cs + kd * plane_t + (size_t)r2 * p.tn_w + SW) * 2);
       x_kd |= (uint32_t)kd << 30;
     }
@@ -248,7 +242,13 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
   struct Staged {
     u32x4 v[ROUNDS];
     uint32_t tail;
-    uint32_t tail_b;  // LEAD only
+    uint32_t tail_b;       // LEAD; EVEN == 0: the dword of the tail's second pixel
+    uint32_t next[ROUNDS];  // EVEN == 0: the dword of the chunk's last pixel
+    uint32_t odd;           // EVEN == 0: one bit per round, the chunk starts on the upper half of a dword; bit 31: the tail
+    // a stage whose windows stick out of the tensors: pixels of the chunks that exist (one bit each, a thread's
+    // chunks all have the same columns), rounds whose row exists (one bit each), pixels of the tail
+    bool masked;
+    uint32_t g_cols, x_cols, rows, tail_cols;
   };
 
   // Loads of one stage into `v`: its two g rows (want_g) and one pair of its x rows
@@ -286,15 +286,17 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     const int hp = cur.hp, ct = cur.ct, od = cur.od, n = cur.n;
     const int oh0 = hp * SR, ow0 = ct * SW;
     const int id0 = od - p.pad_d, ih0 = oh0 - p.pad_h + 2 * xpair, iw0 = ow0 - p.pad_w - LEAD;
-    const char* g_org = reinterpret_cast<const char*>(p.g) +
+    const char* g_org = reinterpret_cast<const char*>(gb) +
                         2 * (((size_t)n * p.cout_total * p.Dout + od) * plane_g + (size_t)oh0 * p.Wout + ow0);
-    const char* x_org = reinterpret_cast<const char*>(p.x) +
+    const char* x_org = reinterpret_cast<const char*>(xb) +
                         2 * ((ptrdiff_t)((size_t)n * p.cin_total * p.Din * plane_x) + (ptrdiff_t)id0 * (ptrdiff_t)plane_x +
                              (ptrdiff_t)ih0 * p.Win + iw0);
     // (with LEAD the window's last dword holds one pixel more than is used; it shares its dword with one that is)
-    const bool inside = ALLIN || (EVEN != 0 && oh0 + SR <= p.Hout && ow0 + SW <= p.Wout && ih0 >= 0 &&
+    const bool inside = ALLIN || (oh0 + SR <= p.Hout && ow0 + SW <= p.Wout && ih0 >= 0 &&
                         ih0 + 2 <= p.Hin && iw0 >= 0 && iw0 + SW + 2 + LEAD <= p.Win && id0 >= 0 &&
-                        id0 + (XC / p.Cin) <= p.Din);
+                        id0 + KD <= p.Din);
+    sg.masked = !inside;
+    sg.odd = 0;
     if (FRAMED && inside) {
       // Rows and columns of the pair's window inside the own tile (wave-uniform): a chunk
       // whose depth plane is a plane of the tile comes from the tile itself, at whatever
@@ -375,59 +377,97 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
 #pragma unroll
       for (int rd = 0; rd < ROUNDS; ++rd) {
         const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;  // THREADS divides G_CHUNKS
-        if (want_g || !g_round) v[rd] = *reinterpret_cast<const u32x4_a4*>((g_round ? g_org : x_org) + c_goff[rd]);
+        if (!want_g && g_round) continue;
+        const uintptr_t at = reinterpret_cast<uintptr_t>(g_round ? g_org : x_org) + c_goff[rd];
+        if (EVEN == 0) {
+          v[rd] = *reinterpret_cast<const u32x4_a4*>(at & ~(uintptr_t)3);
+          sg.next[rd] = *reinterpret_cast<const uint32_t*>((at + 14) & ~(uintptr_t)3);
+          sg.odd |= (uint32_t)((at >> 1) & 1) << rd;
+        } else {
+          v[rd] = *reinterpret_cast<const u32x4_a4*>(at);
+        }
       }
-      sg.tail = *reinterpret_cast<const uint32_t*>(x_org + t_goff);
-      if (LEAD) sg.tail_b = *reinterpret_cast<const uint32_t*>(x_org + t_goff + 4);
+      const uintptr_t at = reinterpret_cast<uintptr_t>(x_org) + t_goff;
+      sg.tail = *reinterpret_cast<const uint32_t*>(at & ~(uintptr_t)3);
+      if (LEAD) sg.tail_b = *reinterpret_cast<const uint32_t*>(at + 4);
+      if (EVEN == 0) {
+        sg.tail_b = *reinterpret_cast<const uint32_t*>((at + 2) & ~(uintptr_t)3);
+        sg.odd |= (uint32_t)((at >> 1) & 1) << 31;
+      }
     } else {
+      // A stage at an edge. A chunk is read wherever its bytes lie inside its tensor, also past the end of its
+      // row; store_loads clears the pixels that are not the row's. A chunk without any pixel of the tensor reads
+      // the workspace instead, so that no load stands under a condition; what is left are the few chunks whose
+      // bytes reach over the tensor's own ends, which go dword by dword.
+      auto columns = [](int col, int count, int cols) {  // of the pixels col .. col + count - 1, those in [0, cols)
+        const int first = max(0, min(count, -col)), past = max(0, min(count, cols - col));
+        return ((1u << past) - 1u) & ~((1u << first) - 1u);
+      };
+      const int c8 = tid & 7;  // a round is a multiple of 8 chunks: the same in all of them
+      sg.g_cols = columns(ow0 + c8 * 8, 8, p.Wout);
+      sg.x_cols = columns(iw0 + c8 * 8, 8, p.Win);
+      sg.rows = 0;
+      uint32_t over = 0;
 #pragma unroll
       for (int rd = 0; rd < ROUNDS; ++rd) {
+        const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;
+        if (!want_g && g_round) continue;
         const int q = tid + rd * THREADS;
-        u32x4 val = {0u, 0u, 0u, 0u};
-        if (q < CHUNKS && (want_g || q >= G_CHUNKS)) {
-          const bool is_x = q >= G_CHUNKS;
-          const uint16_t* src;
-          int row, col, rows, cols;
-          bool ok = true;
-          if (!is_x) {
-            const int c8 = q & 7, r = (q >> 3) % SR;
-            src = reinterpret_cast<const uint16_t*>(g_org + c_goff[rd]);
-            row = oh0 + r; col = ow0 + c8 * 8; rows = p.Hout; cols = p.Wout;
-          } else {
-            const int qx = q - G_CHUNKS;
-            const int c8 = qx % X_CPR, rr = qx / X_CPR;
-            const int r2 = rr & 1, ch = rr >> 1;
-            src = reinterpret_cast<const uint16_t*>(x_org + c_goff[rd]);
-            row = ih0 + r2; col = iw0 + c8 * 8; rows = p.Hin; cols = p.Win;
-            const int dd = id0 + ch / p.Cin;
-            ok = dd >= 0 && dd < p.Din;
-          }
-          if (ok && row >= 0 && row < rows) {
-            if (col >= 0 && col + 8 <= cols && (reinterpret_cast<uintptr_t>(src) & 3) == 0) {
-              val = *reinterpret_cast<const u32x4_a4*>(src);
-            } else {
-              uint32_t e[8];
+        bool row_ok;
+        if (g_round) {
+          row_ok = oh0 + ((q >> 3) % SR) < p.Hout;
+        } else {
+          const int rr = (q - G_CHUNKS) / X_CPR;
+          const int row = ih0 + (rr & 1), dd = id0 + (rr >> 1) / CIN_B;
+          row_ok = q < CHUNKS && row >= 0 && row < p.Hin && dd >= 0 && dd < p.Din;
+        }
+        const bool need = row_ok && (g_round ? sg.g_cols : sg.x_cols) != 0u;
+        sg.rows |= (need ? 1u : 0u) << rd;
+        const char* a = (g_round ? g_org : x_org) + c_goff[rd];
+        const bool fits = a >= reinterpret_cast<const char*>(g_round ? p.g : p.x) && a + 16 <= (g_round ? p.g_end : p.x_end);
+        over |= (need && !fits ? 1u : 0u) << rd;
+        const uintptr_t at = reinterpret_cast<uintptr_t>(need && fits ? a : reinterpret_cast<const char*>(p.part));
+        v[rd] = *reinterpret_cast<const u32x4_a4*>(at & ~(uintptr_t)3);
+        if (EVEN == 0) {
+          sg.next[rd] = *reinterpret_cast<const uint32_t*>((at + 14) & ~(uintptr_t)3);
+          sg.odd |= (uint32_t)((at >> 1) & 1) << rd;
+        }
+      }
+      auto dword_at = [](uintptr_t at, const void* begin, const char* end) {  // 0 where it holds no pixel of the tensor
+        return at + 4 > reinterpret_cast<uintptr_t>(begin) && at < reinterpret_cast<uintptr_t>(end) ? *reinterpret_cast<const uint32_t*>(at) : 0u;
+      };
+      if (__builtin_amdgcn_ballot_w64(over != 0u) != 0) {
 #pragma unroll
-              for (int k = 0; k < 8; ++k) e[k] = (col + k >= 0 && col + k < cols) ? (uint32_t)src[k] : 0u;
-              val.x = e[0] | (e[1] << 16); val.y = e[2] | (e[3] << 16);
-              val.z = e[4] | (e[5] << 16); val.w = e[6] | (e[7] << 16);
-            }
+        for (int rd = 0; rd < ROUNDS; ++rd) {
+          if (((over >> rd) & 1u) == 0) continue;
+          const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;
+          const void* begin = g_round ? p.g : p.x;
+          const char* end = g_round ? p.g_end : p.x_end;
+          const uintptr_t at = reinterpret_cast<uintptr_t>((g_round ? g_org : x_org) + c_goff[rd]);
+          const uintptr_t down = at & ~(uintptr_t)3;
+          v[rd].x = dword_at(down, begin, end);
+          v[rd].y = dword_at(down + 4, begin, end);
+          v[rd].z = dword_at(down + 8, begin, end);
+          v[rd].w = dword_at(down + 12, begin, end);
+          if (EVEN == 0) {
+            sg.next[rd] = dword_at((at + 14) & ~(uintptr_t)3, begin, end);
+            sg.odd = (sg.odd & ~(1u << rd)) | ((uint32_t)((at >> 1) & 1) << rd);
           }
         }
-        v[rd] = val;
       }
       if (has_tail) {
         const int r2 = tid & 1, ch = tid >> 1;
-        const int row = ih0 + r2, col = iw0 + SW, dd = id0 + ch / p.Cin;
-        const uint16_t* src = reinterpret_cast<const uint16_t*>(x_org + t_goff);
-        uint32_t e[4] = {0u, 0u, 0u, 0u};
-        if (dd >= 0 && dd < p.Din && row >= 0 && row < p.Hin) {
-#pragma unroll
-          for (int k = 0; k < 2 + 2 * LEAD; ++k)
-            if (col + k >= 0 && col + k < p.Win) e[k] = src[k];
+        const int row = ih0 + r2, dd = id0 + ch / CIN_B;
+        const uintptr_t at = reinterpret_cast<uintptr_t>(x_org) + t_goff;
+        const uintptr_t down = at & ~(uintptr_t)3;
+        const bool ok = dd >= 0 && dd < p.Din && row >= 0 && row < p.Hin;
+        sg.tail_cols = ok ? columns(iw0 + SW, 2 + 2 * LEAD, p.Win) : 0u;
+        sg.tail = sg.tail_cols != 0u ? dword_at(down, p.x, p.x_end) : 0u;
+        if (LEAD) sg.tail_b = (sg.tail_cols >> 2) != 0u ? dword_at(down + 4, p.x, p.x_end) : 0u;
+        if (EVEN == 0) {
+          sg.tail_b = sg.tail_cols != 0u ? dword_at((at + 2) & ~(uintptr_t)3, p.x, p.x_end) : 0u;
+          sg.odd |= (uint32_t)((at >> 1) & 1) << 31;
         }
-        sg.tail = e[0] | (e[1] << 16);
-        sg.tail_b = e[2] | (e[3] << 16);
       }
     }
   };
@@ -438,24 +478,52 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
 #pragma unroll
   for (int rd = 0; rd < ROUNDS; ++rd) bsum[rd] = 0.0f;
   auto store_loads = [&](const Staged& sg, bool have_g, int gbuf, int slot_a, int slot_b, bool counted = true) {
-    const u32x4 (&v)[ROUNDS] = sg.v;
+    uint32_t g_keep[4], x_keep[4];
+    if (!ALLIN && sg.masked) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        g_keep[j] = (((sg.g_cols >> (2 * j)) & 1u) * 0xffffu) | (((sg.g_cols >> (2 * j + 1)) & 1u) * 0xffff0000u);
+        x_keep[j] = (((sg.x_cols >> (2 * j)) & 1u) * 0xffffu) | (((sg.x_cols >> (2 * j + 1)) & 1u) * 0xffff0000u);
+      }
+    }
 #pragma unroll
     for (int rd = 0; rd < ROUNDS; ++rd) {
       const int q = tid + rd * THREADS;
-      if (q < G_CHUNKS) {
-        if (have_g) {
-          *reinterpret_cast<u32x4*>(smem + gbuf * G_BYTES + c_lds[rd]) = v[rd];
-          if (p.bias_part != nullptr) bsum[rd] += counted ? sum_bf16x8(v[rd]) : 0.0f;
-        }
+      const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;
+      if (g_round && !have_g) continue;
+      u32x4 val = sg.v[rd];
+      if (EVEN == 0) {
+        const uint32_t shift = ((sg.odd >> rd) & 1u) << 4;
+        val.x = __builtin_amdgcn_alignbit(val.y, val.x, shift);
+        val.y = __builtin_amdgcn_alignbit(val.z, val.y, shift);
+        val.z = __builtin_amdgcn_alignbit(val.w, val.z, shift);
+        val.w = __builtin_amdgcn_alignbit(sg.next[rd], val.w, shift);
+      }
+      if (!ALLIN && sg.masked) {  // uniform
+        const uint32_t row = 0u - ((sg.rows >> rd) & 1u);
+        val.x &= (g_round ? g_keep[0] : x_keep[0]) & row;
+        val.y &= (g_round ? g_keep[1] : x_keep[1]) & row;
+        val.z &= (g_round ? g_keep[2] : x_keep[2]) & row;
+        val.w &= (g_round ? g_keep[3] : x_keep[3]) & row;
+      }
+      if (g_round) {
+        *reinterpret_cast<u32x4*>(smem + gbuf * G_BYTES + c_lds[rd]) = val;
+        if (bias_part != nullptr) bsum[rd] += counted ? sum_of_8<F16>(val) : 0.0f;
       } else if (q < CHUNKS) {
         const int slot = ((x_second >> rd) & 1u) ? slot_b : slot_a;
-        *reinterpret_cast<u32x4*>(lds_x + c_lds[rd] + slot * X_ROW) = v[rd];
+        *reinterpret_cast<u32x4*>(lds_x + c_lds[rd] + slot * X_ROW) = val;
       }
     }
     if (has_tail) {
       unsigned char* at = lds_x + t_lds + ((tid & 1) ? slot_b : slot_a) * X_ROW;
-      *reinterpret_cast<uint32_t*>(at) = sg.tail;
-      if (LEAD) *reinterpret_cast<uint32_t*>(at + 4) = sg.tail_b;
+      uint32_t t = sg.tail, tb = sg.tail_b;
+      if (EVEN == 0) t = __builtin_amdgcn_alignbit(tb, t, (sg.odd >> 31) << 4);
+      if (!ALLIN && sg.masked) {
+        t &= ((sg.tail_cols & 1u) * 0xffffu) | (((sg.tail_cols >> 1) & 1u) * 0xffff0000u);
+        if (LEAD) tb &= (((sg.tail_cols >> 2) & 1u) * 0xffffu) | (((sg.tail_cols >> 3) & 1u) * 0xffff0000u);
+      }
+      *reinterpret_cast<uint32_t*>(at) = t;
+      if (LEAD) *reinterpret_cast<uint32_t*>(at + 4) = tb;
     }
   };
 
@@ -644,7 +712,8 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
   }
 
   // bias partial of this workgroup: the 16 lanes that carried a channel's chunks add up
-  if (p.bias_part != nullptr) {
+  const size_t slot = (size_t)block * gridDim.x + blockIdx.x;
+  if (bias_part != nullptr) {
 #pragma unroll
     for (int rd = 0; rd < ROUNDS; ++rd) {
       const int q = tid + rd * THREADS;
@@ -654,80 +723,131 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
         s += __shfl_xor(s, 4, 64);
         s += __shfl_xor(s, 2, 64);
         s += __shfl_xor(s, 1, 64);
-        if (q < G_CHUNKS && (tid & 15) == 0) p.bias_part[(size_t)blockIdx.x * GC + q / (8 * SR)] = s;
+        if (q < G_CHUNKS && (tid & 15) == 0) bias_part[slot * GC + q / (8 * SR)] = s;
       }
     }
   }
 
-  // partial of this wavefront: slot = workgroup * HALVES + half, layout [tap9][co][c']
-  if (wave >= CWAVES) return;
-  float* out = p.part + ((size_t)blockIdx.x * HALVES + half) * (size_t)(9 * GC * XC);
+  // Partial of this workgroup. The two column halves of a pair meet in LDS first (the stage buffers are free:
+  // a barrier closed the last stage), three taps at a time, which halves what goes to memory and comes back.
+  // A lane's 16 values of a tap leave as four 16-byte pieces, [tap9][pair][4][lane][4].
+  static_assert(CGB * CXB * 3 * 4096 <= 2 * G_BYTES + XC * X_CH, "three taps of every pair fit the stage buffers");
+  float* const meet = reinterpret_cast<float*>(smem) + pair * 3 * 1024 + lane * 4;
+  float* const out = p.part + slot * (size_t)(9 * GC * XC) + pair * 1024 + lane * 4;
 #pragma unroll
-  for (int kh = 0; kh < 3; ++kh)
+  for (int kh = 0; kh < 3; ++kh) {
+    if (wave < CWAVES && half == 1) {
 #pragma unroll
-    for (int kw = 0; kw < 3; ++kw)
+      for (int kw = 0; kw < 3; ++kw)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int co = cb * 32 + 8 * (i >> 2) + 4 * kgp + (i & 3);
-        out[((kh * 3 + kw) * GC + co) * XC + ib * 32 + ln] = acc[kh][kw][i];
-      }
+        for (int j = 0; j < 4; ++j)
+          *reinterpret_cast<f32x4*>(meet + kw * 1024 + j * 256) =
+              f32x4{acc[kh][kw][4 * j], acc[kh][kw][4 * j + 1], acc[kh][kw][4 * j + 2], acc[kh][kw][4 * j + 3]};
+    }
+    __syncthreads();
+    if (wave < CWAVES && half == 0) {
+#pragma unroll
+      for (int kw = 0; kw < 3; ++kw)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          f32x4 v = *reinterpret_cast<const f32x4*>(meet + kw * 1024 + j * 256);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) v[k] += acc[kh][kw][4 * j + k];
+          *reinterpret_cast<f32x4*>(out + (size_t)(kh * 3 + kw) * (GC * XC) + j * 256) = v;
+        }
+    }
+    __syncthreads();
+  }
 }
 
-// gb[co] (bf16) = sum over the workgroups of bias_part[wg][co]; one wavefront per channel,
-// fixed order. GC = channels per partial row, `valid` of them exist.
-__global__ __launch_bounds__(256) void wgrad_bias_reduce_kernel(uint16_t* __restrict__ gb,
-                                                                const float* __restrict__ part,
-                                                                int wgs, int GC, int valid) {
-  const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (c >= valid) return;
-  float s = 0.0f;
-  for (int k = lane; k < wgs; k += 64) s += part[(size_t)k * GC + c];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if (lane == 0) gb[c] = jg::f32_to_bf16(s);
+// gw = sum over the partials of a block of channels (its workgroups, and in split mode its part pairs, which
+// lie behind each other), and gb the same over the bias partials. A workgroup owns one run of 256 values of a
+// block's partial (a tap, a pair, four registers), a lane four of them; its 8 wavefronts take every eighth
+// partial in chains of their own and the sums are added in a fixed order (deterministic). What bounds it is
+// the latency of the chains: 16-byte loads, eight in flight per lane.
+// The workgroups behind those of the last block add up bias partials, one lane per channel.
+struct ReduceParams {
+  const float* part;
+  const float* bias_part;
+  void* gw;
+  void* gb;
+  int wgs, npairs;            // workgroups of a block, part pairs
+  int pairs, GC, CXB, cin_b;  // 32 x 32 pairs of a block; its g channels, x blocks and x channels per depth tap
+  int KD, cin, cout, ci_blocks;
+  int gw_blocks;              // workgroups that reduce gw
+  int bias_cout, bias_parts;  // output channels, and parts of g whose bias sums belong together
+};
+constexpr int RED_WAVES = 8;
+template <int OUT>  // dtype of gw and gb: 0 bf16, 1 fp32, 2 fp16
+__device__ __forceinline__ void store_gradient(void* out, size_t at, float v) {
+  if (OUT == 1) static_cast<float*>(out)[at] = v;
+  else if (OUT == 2) static_cast<_Float16*>(out)[at] = (_Float16)v;
+  else static_cast<uint16_t*>(out)[at] = jg::f32_to_bf16(v);
 }
-
-// gw[co0 + co][ci0 + ci][kd][kh][kw] (bf16) = sum over the slots of
-// part[slot][tap9][co][kd*CinB+ci] for the channels of the block that exist (gw points at
-// the block's first element, cin_total is the channel count of the whole weight tensor).
-// A block owns 64 consecutive outputs (one per lane, so a slot row is read coalesced);
-// its 4 wavefronts take the slots s = w, w + 4, ... in 4 independent chains each, and the
-// 16 chain sums are added in a fixed order (deterministic).
-template <bool OUT32>
-__global__ __launch_bounds__(256) void wgrad_reduce_kernel(void* __restrict__ gw_out,
-                                                           const float* __restrict__ part,
-                                                           int slots, int GC, int XC, int CinB,
-                                                           int cout_valid, int cin_valid, int cin_total, int accumulate) {
-  __shared__ float red[4][64];
-  const int count = 9 * GC * XC;
+template <int OUT>
+__global__ __launch_bounds__(64 * RED_WAVES) void wgrad_reduce_kernel(ReduceParams p) {
+  __shared__ f32x4 red[RED_WAVES][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int i = blockIdx.x * 64 + lane;  // index in [tap9][co][c']
-  float c0 = 0.f, c1 = 0.f, c2 = 0.f, c3 = 0.f;
-  if (i < count) {
-    int k = w;
-    for (; k + 12 < slots; k += 16) {
-      c0 += part[(size_t)(k + 0) * count + i];
-      c1 += part[(size_t)(k + 4) * count + i];
-      c2 += part[(size_t)(k + 8) * count + i];
-      c3 += part[(size_t)(k + 12) * count + i];
+  if ((int)blockIdx.x >= p.gw_blocks) {
+    // bias: 64 channels per workgroup; a channel's block at x block 0 and x part 0 holds its sums
+    const int c = ((int)blockIdx.x - p.gw_blocks) * 64 + lane;
+    float s = 0.0f;
+    if (c < p.bias_cout) {
+      for (int gp = p.bias_parts - 1; gp >= 0; --gp) {
+        // plain: one pair per block. Part pairs: the pair (gp, 0) is pair kBias of the block
+        const int pair_k = p.npairs == 6 ? (gp == 2 ? 2 : (gp == 1 ? 4 : 5)) : 0;
+        const int row = p.npairs == 1 ? gp * p.bias_cout + c : c;  // all parts in one block: parts are channels of it
+        const size_t slot0 = ((size_t)(row / p.GC) * p.ci_blocks * p.npairs + pair_k) * p.wgs;
+        const float* src = p.bias_part + slot0 * p.GC + row % p.GC;
+        float c8[8] = {};
+        for (int k = w; k < p.wgs; k += 8 * RED_WAVES) {
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const int at = k + u * RED_WAVES;
+            c8[u] += at < p.wgs ? src[(size_t)at * p.GC] : 0.0f;
+          }
+        }
+        s += ((c8[0] + c8[1]) + (c8[2] + c8[3])) + ((c8[4] + c8[5]) + (c8[6] + c8[7]));
+      }
     }
-    for (; k < slots; k += 4) c0 += part[(size_t)k * count + i];
+    red[w][lane].x = s;
+    __syncthreads();
+    if (w != 0 || c >= p.bias_cout) return;
+    s = 0.0f;
+#pragma unroll
+    for (int k = 0; k < RED_WAVES; ++k) s += red[k][lane].x;
+    store_gradient<OUT>(p.gb, c, s);
+    return;
   }
-  red[w][lane] = (c0 + c1) + (c2 + c3);
+  const int runs = 9 * p.pairs * 4;  // runs of 256 values in a block's partial
+  const int blk = blockIdx.x / runs, run = blockIdx.x - blk * runs;
+  const int slots = p.wgs * p.npairs;
+  const size_t stride = (size_t)runs * 256;
+  const float* src = p.part + (size_t)blk * slots * stride + (size_t)run * 256 + lane * 4;
+  f32x4 c[8] = {};
+  int k = w;
+  for (; k + 7 * RED_WAVES < slots; k += 8 * RED_WAVES) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) c[u] += *reinterpret_cast<const f32x4*>(src + (size_t)(k + u * RED_WAVES) * stride);
+  }
+#pragma unroll
+  for (int u = 0; u < 7; ++u)
+    if (k + u * RED_WAVES < slots) c[u] += *reinterpret_cast<const f32x4*>(src + (size_t)(k + u * RED_WAVES) * stride);
+  red[w][lane] = ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
   __syncthreads();
-  if (w != 0 || i >= count) return;
-  const float s = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
-  const int cx = i % XC, co = (i / XC) % GC, tap = i / (XC * GC);
-  const int kd = cx / CinB, ci = cx % CinB, KD = XC / CinB;
-  if (co >= cout_valid || ci >= cin_valid) return;
-  const size_t at = (((size_t)co * cin_total + ci) * KD + kd) * 9 + tap;
-  if (OUT32) {
-    // split mode: the six part products of a block are added up here, one launch after the other
-    float* gw = static_cast<float*>(gw_out);
-    gw[at] = accumulate ? gw[at] + s : s;
-  } else {
-    static_cast<uint16_t*>(gw_out)[at] = jg::f32_to_bf16(s);
+  if (w != 0) return;
+  f32x4 sum = red[0][lane];
+#pragma unroll
+  for (int u = 1; u < RED_WAVES; ++u) sum += red[u][lane];
+  const int j = run & 3, pair = (run >> 2) % p.pairs, tap = (run >> 2) / p.pairs;
+  const int cb = pair / p.CXB, ib = pair % p.CXB;
+  const int cx = ib * 32 + (lane & 31), kd = cx / p.cin_b;
+  const int ci = (blk % p.ci_blocks) * p.cin_b + cx % p.cin_b;
+  if (ci >= p.cin) return;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int co = (blk / p.ci_blocks) * p.GC + cb * 32 + 8 * j + 4 * (lane >> 5) + u;
+    if (co < p.cout) store_gradient<OUT>(p.gw, (((size_t)co * p.cin + ci) * p.KD + kd) * 9 + tap, sum[u]);
   }
 }
 
@@ -747,11 +867,6 @@ __global__ __launch_bounds__(256) void wgrad_combine_parts_kernel(float* __restr
   gw[idx] = sum;
 }
 
-__global__ __launch_bounds__(256) void f32_to_f16_kernel(_Float16* __restrict__ dst, const float* __restrict__ src, int n) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) dst[i] = (_Float16)src[i];
-}
-
 int cu_count() {
   static int cached = 0;
   if (cached) return cached;
@@ -763,52 +878,70 @@ int cu_count() {
   return n;
 }
 
-int wg_count(long long stages) {
-  long long n = cu_count();
-  if (n > stages) n = stages;
-  if (n < 1) n = 1;
-  return (int)n;
-}
-
 long long stage_count(const ConvGeom& g) {
   return g.batch * g.out[0] * ((g.out[1] + SR - 1) / SR) * ((g.out[2] + SW - 1) / SW);
 }
 
-// (CGB, CXB) of a geometry, or false when the kernel does not cover it
-// Channel blocking. One launch accumulates a block of `cob` output x `cib` input channels
-// (32 or 64 each; with a depth kernel of 3 always 32 x 32, so that the x side spans 96);
-// more channels are covered block by block, a last block with fewer channels than its
-// width re-reads its last channel and its extra rows and columns are dropped.
-struct Blocking {
-  int cob, cib;  // width of the first (largest) block
-  int KD;
-  int cob_max() const { return KD == 3 ? 32 : 64; }
-  int cib_max() const { return KD == 3 ? 32 : 64; }
+// Channel blocking. A workgroup accumulates a block of GC output x CIN_B input channels (32 or 64 each; with a
+// depth kernel of 3 always 32 x 32, so that the x side spans 96); a block with fewer channels than its width
+// re-reads its last channel and its extra rows and columns are dropped. All blocks of a problem run in one
+// launch: one launch each (with its own reduction) took 269 us where this takes 97, 119 -> 191 channels of 4 x 74 x 88.
+struct Plan {
+  int cgb, cxb, KD;
+  int co_blocks, ci_blocks, npairs;
+  int parts_in_block;  // split mode: parts that are channels of the one block (1: the parts are block pairs)
+  int wgs;             // workgroups per block
+  size_t GC() const { return 32 * cgb; }
+  size_t XC() const { return 32 * cxb; }
+  size_t blocks() const { return (size_t)co_blocks * ci_blocks * npairs; }
+  size_t partial() const { return 9 * GC() * XC(); }  // floats
+  size_t bytes() const { return (blocks() * wgs * (partial() + GC()) * sizeof(float) + 255) / 256 * 256; }
 };
-bool blocks_of(const ConvGeom& g, Blocking* b) {
+bool covered(const ConvGeom& g) {
   if (g.groups != 1) return false;
   if (g.k[1] != 3 || g.k[2] != 3 || (g.k[0] != 1 && g.k[0] != 3)) return false;
   if (g.k[0] == 1 && g.in[0] != 1) return false;
   for (int a = 0; a < 3; ++a)
     if (g.s[a] != 1 || g.d[a] != 1) return false;
   if (g.cin <= 0 || g.cout <= 0) return false;
-  b->KD = g.k[0];
-  if (b->KD == 3) {
-    b->cob = 32; b->cib = 32;
-  } else {
-    b->cob = g.cout > 32 ? 64 : 32;
-    b->cib = g.cin > 32 ? 64 : 32;
-  }
   // per-lane byte offsets inside one batch entry are 32-bit
   const size_t xs = (size_t)g.cin * g.in[0] * g.in[1] * g.in[2] * 2;
   const size_t gs = (size_t)g.cout * g.out[0] * g.out[1] * g.out[2] * 2;
   return xs < (1ull << 31) && gs < (1ull << 31);
 }
-// width of the block that starts at channel c0 of `total`
-int block_width(int total, int c0, int first) { return (first == 64 && total - c0 > 32) ? 64 : 32; }
+Plan plan_of(const ConvGeom& g, int parts) {
+  Plan p;
+  p.KD = g.k[0];
+  const int widest = p.KD == 3 ? 32 : 64;
+  p.parts_in_block = parts > 1 && parts * g.cout <= widest && parts * g.cin <= widest ? parts : 1;
+  const int cout = p.parts_in_block * g.cout, cin = p.parts_in_block * g.cin;
+  // 64 channels a side where that pads no further than 32 would: the wider block reads its operands for twice
+  // the products
+  auto width = [&](int c) { return widest == 64 && (c + 63) / 64 * 64 <= (c + 31) / 32 * 32 ? 64 : 32; };
+  const int cob = width(cout), cib = width(cin);
+  p.cgb = cob / 32;
+  p.cxb = p.KD * cib / 32;
+  p.co_blocks = (cout + cob - 1) / cob;
+  p.ci_blocks = (cin + cib - 1) / cib;
+  p.npairs = parts > 1 && p.parts_in_block == 1 ? 6 : 1;
+  // Workgroups per block. More of them shorten the walk over the pixels and lengthen the reduction of their
+  // partials: a walk of `stages` at about 2 us each (a 64 x 64 block; a smaller one waits as long for its loads)
+  // against partials that are written and read at about 4 TB/s, W = sqrt(stages * 2 us * 4 TB/s / 2 / bytes)
+  // workgroups in all; not more than the chip holds at once, and whole XCD rounds where there are that many.
+  const long long stages = stage_count(g);
+  const double blocks = (double)p.blocks(), bytes = (double)p.partial() * sizeof(float);
+  const double best = sqrt((double)stages * blocks * 4.0e6 / bytes);
+  const double most = cu_count() * (p.cgb * p.cxb == 1 ? 2.0 : 1.0);
+  long long n = (long long)((best < most ? best : most) / blocks);
+  if (n >= 8) n = n / 8 * 8;
+  if (n > stages) n = stages;
+  if (n < 1) n = 1;
+  p.wgs = (int)n;
+  return p;
+}
 
 template <int CGB, int CXB>
-int launch(const WgradParams& p, int even, bool f16, bool all_inside, int wgs, hipStream_t s, const char* who) {
+int launch(const WgradParams& p, int even, bool f16, bool all_inside, dim3 grid, hipStream_t s, const char* who) {
   constexpr int THREADS = wgrad_threads(CGB, CXB);
   const size_t lds = 2 * (size_t)(32 * CGB * G_CH) + (size_t)(32 * CXB * X_CH);
   void (*kern)(WgradParams);
@@ -825,7 +958,7 @@ int launch(const WgradParams& p, int even, bool f16, bool all_inside, int wgs, h
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %zu bytes of LDS", who, lds);
-  kern<<<wgs, THREADS, lds, s>>>(p);
+  kern<<<grid, THREADS, lds, s>>>(p);
   return JG_OK;
 }
 
@@ -835,47 +968,23 @@ namespace jg {
 
 // fp32 is split into three bf16 parts per operand; fp16 has its own MFMA instruction and runs like bf16
 static int parts_of(int dtype) { return dtype == JG_F32 ? 3 : 1; }
-// Split mode with few channels: the parts of both operands fit one block.
-static bool parts_fit_one_block(const ConvGeom& g, const Blocking& bl, int parts) {
-  return parts > 1 && parts * g.cout <= bl.cob_max() && parts * g.cin <= bl.cib_max();
-}
-static size_t parts_tmp_bytes(const ConvGeom& g, const Blocking& bl, int parts) {
-  if (!parts_fit_one_block(g, bl, parts)) return 0;
-  return ((size_t)parts * parts * g.cout * g.cin * bl.KD * 9 * sizeof(float) + 255) / 256 * 256;
-}
-// fp16: the gradient is reduced into fp32 here before the one rounding to fp16
-static size_t acc32_bytes(const ConvGeom& g, int dtype) {
-  return dtype == JG_F16 ? ((size_t)g.cout * g.cin * g.k[0] * 9 * sizeof(float) + 255) / 256 * 256 : 0;
-}
-
 // fp32 runs in split mode: both operands are copied as three bf16 parts each (as extra channels) and
 // the six part products whose indices add up to at most 2 are accumulated in fp32.
 bool mfma_wgrad_supported(const ConvGeom& g, int dtype) {
-  Blocking b;
   if ((dtype != JG_BF16 && dtype != JG_F32 && dtype != JG_F16) || g.batch <= 0) return false;
-  return blocks_of(g, &b);
+  return covered(g);
 }
 
-static size_t partial_bytes(const ConvGeom& g) {
-  Blocking b{32, 32, 1};
-  blocks_of(g, &b);
-  const size_t wgs = (size_t)wg_count(stage_count(g));
-  // sized for the widest block any mode launches
-  const size_t n = wgs * HALVES * 9 * b.cob_max() * (b.KD * b.cib_max()) * sizeof(float) + wgs * b.cob_max() * sizeof(float);
-  return (n + 255) / 256 * 256;
-}
 static size_t split_copy_bytes(size_t elements, int parts) { return (elements * parts * 2 + 255) / 256 * 256; }
-// workspace: [partials | fp32 sum (fp16 only) | x parts | g parts (fp32 only) | part products of the one-block launch]
+// workspace: [partials | x parts | g parts (fp32 only) | part products of the one-block launch]
 size_t mfma_wgrad_workspace(const ConvGeom& g, int dtype) {
-  size_t n = partial_bytes(g);
   const int parts = parts_of(dtype);
-  n += acc32_bytes(g, dtype);  // fp16 only, directly behind the partial sums
+  const Plan plan = plan_of(g, parts);
+  size_t n = plan.bytes();
   if (parts > 1) {
     n += split_copy_bytes((size_t)g.batch * g.cin * g.in[0] * g.in[1] * g.in[2], parts);
     n += split_copy_bytes((size_t)g.batch * g.cout * g.out[0] * g.out[1] * g.out[2], parts);
-    Blocking b{32, 32, 1};
-    blocks_of(g, &b);
-    n += parts_tmp_bytes(g, b, parts);
+    if (plan.parts_in_block > 1) n += ((size_t)parts * parts * g.cout * g.cin * plan.KD * 9 * sizeof(float) + 255) / 256 * 256;
   }
   return n;
 }
@@ -885,8 +994,9 @@ size_t mfma_wgrad_workspace(const ConvGeom& g, int dtype) {
 // inside the bands that the frame holds.
 bool mfma_wgrad_frame_ok(const ConvGeom& g, const int tlo[3], const int tn[3]) {
   if (g.in[2] % 2 != 0 || g.p[2] % 2 != 0 || g.out[2] % 2 != 0 || tn[2] % 2 != 0) return false;
-  Blocking b;  // the framed input is read by a single block of exactly its width
-  if (!blocks_of(g, &b) || g.cin != b.cib || g.cout != b.cob) return false;
+  if (!covered(g)) return false;
+  const Plan plan = plan_of(g, 1);  // the framed input is read by a single block of exactly its width
+  if (g.cin * plan.KD != (int)plan.XC() || g.cout != (int)plan.GC()) return false;
   int blo[3], bhi[3];
   mfma_frame_bands(g, tlo, tn, blo, bhi);
   const int row_pairs = (g.out[1] + SR - 1) / SR, col_tiles = (g.out[2] + SW - 1) / SW;
@@ -910,8 +1020,7 @@ bool mfma_wgrad_frame_ok(const ConvGeom& g, const int tlo[3], const int tn[3]) {
 int mfma_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom& g, void* ws,
                size_t ws_bytes, hipStream_t s, const void* xt, const int* tlo, const int* tn, int dtype) {
   const char* who = "jg_conv_wgrad(mfma)";
-  Blocking bl;
-  if (!blocks_of(g, &bl)) JG_FAIL(JG_ERR_UNSUPPORTED, "%s: geometry not covered", who);
+  if (!covered(g)) JG_FAIL(JG_ERR_UNSUPPORTED, "%s: geometry not covered", who);
   if (ws == nullptr || ws_bytes < mfma_wgrad_workspace(g, dtype))
     JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, ws_bytes,
             mfma_wgrad_workspace(g, dtype));
@@ -919,15 +1028,12 @@ int mfma_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom
              who);
   const size_t x_cs = (size_t)g.in[0] * g.in[1] * g.in[2], g_cs = (size_t)g.out[0] * g.out[1] * g.out[2];
   const int parts = parts_of(dtype);
-  const bool split = parts > 1;
+  const Plan plan = plan_of(g, parts);
   const bool f16 = dtype == JG_F16;
-  float* sum32 = static_cast<float*>(gw);  // where the part products are added up (split mode)
   float* one_block_tmp = nullptr;
-  if ((split || f16) && (gb != nullptr || xt != nullptr))
-    JG_FAIL(JG_ERR_UNSUPPORTED, "%s: fp32 / fp16 have neither the fused bias gradient nor the framed input", who);
-  if (f16) sum32 = reinterpret_cast<float*>(static_cast<char*>(ws) + partial_bytes(g));
-  if (split) {
-    char* base = static_cast<char*>(ws) + partial_bytes(g);
+  if (dtype != JG_BF16 && xt != nullptr) JG_FAIL(JG_ERR_UNSUPPORTED, "%s: the framed input is bf16", who);
+  if (parts > 1) {
+    char* base = static_cast<char*>(ws) + plan.bytes();
     uint16_t* xs = reinterpret_cast<uint16_t*>(base);
     base += split_copy_bytes((size_t)g.batch * g.cin * x_cs, parts);
     uint16_t* gs = reinterpret_cast<uint16_t*>(base);
@@ -946,120 +1052,66 @@ int mfma_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom
   const int even = !even_rows ? 0 : (g.p[2] % 2 == 0 ? 1 : 2);
   if (xt != nullptr && (even != 1 || !mfma_wgrad_frame_ok(g, tlo, tn)))
     JG_FAIL(JG_ERR_UNSUPPORTED, "%s: the framed input does not cover this geometry / alignment", who);
-  // part products (g part, x part), smallest first; plain mode: the one product
-  static const int kPairs[6][2] = {{0, 2}, {1, 1}, {2, 0}, {0, 1}, {1, 0}, {0, 0}};
-  const int npairs = parts == 3 ? 6 : (parts == 2 ? 3 : 1), first_pair = 6 - npairs;
-  const int gw_count = g.cout * g.cin * g.k[0] * 9;
-  auto finish = [&]() -> int {  // fp16: the one rounding of the fp32 sum
-    if (dtype == JG_F16) {
-      f32_to_f16_kernel<<<(gw_count + 255) / 256, 256, 0, s>>>(static_cast<_Float16*>(gw), sum32, gw_count);
-      JG_CHECK_LAUNCH(who);
-    }
-    return JG_OK;
-  };
   WgradParams p;
   p.part = static_cast<float*>(ws);
+  p.bias_part = gb != nullptr ? p.part + plan.blocks() * plan.wgs * plan.partial() : nullptr;
+  p.x = static_cast<const uint16_t*>(x);
+  p.g = static_cast<const uint16_t*>(go);
   p.x_end = static_cast<const char*>(x) + 2 * (size_t)g.batch * parts * g.cin * x_cs;
+  p.g_end = static_cast<const char*>(go) + 2 * (size_t)g.batch * parts * g.cout * g_cs;
+  p.cin = plan.parts_in_block * g.cin; p.cout = plan.parts_in_block * g.cout;
   p.cin_total = parts * g.cin; p.cout_total = parts * g.cout;
+  p.ci_blocks = plan.ci_blocks; p.npairs = plan.npairs;
+  // part products (g part, x part), smallest first; plain mode: the one product
+  p.gparts = plan.npairs == 6 ? 0u | (1u << 2) | (2u << 4) | (0u << 6) | (1u << 8) | (0u << 10) : 0u;
+  p.xparts = plan.npairs == 6 ? 2u | (1u << 2) | (0u << 4) | (1u << 6) | (0u << 8) | (0u << 10) : 0u;
   p.Din = g.in[0]; p.Hin = g.in[1]; p.Win = g.in[2];
   p.Dout = g.out[0]; p.Hout = g.out[1]; p.Wout = g.out[2];
   p.pad_d = g.p[0]; p.pad_h = g.p[1]; p.pad_w = g.p[2];
   p.row_pairs = (g.out[1] + SR - 1) / SR;
   p.col_tiles = (g.out[2] + SW - 1) / SW;
   p.total_stages = stage_count(g);
-  {
-    // column strips outside the kernel's vector-load path (see the kernel's `inside`)
-    const int last_ow0 = (p.col_tiles - 1) * SW;
-    const bool first_slow = g.p[2] > 0;
-    const int lead = even == 2 ? 1 : 0;
-    const bool last_slow = last_ow0 + SW > g.out[2] || last_ow0 - g.p[2] - lead + SW + 2 + lead > g.in[2];
-    p.w_first = p.w_last = p.wd_first = p.wd_last = 1;
-    // measured: such a stage costs about four plain ones; 3 gave the shortest kernels over the shapes tried
-    constexpr int SLOW = 3;
-    if (even) {  // without the even layout every stage takes that path
-      if (p.col_tiles == 1) p.w_first = (first_slow || last_slow) ? SLOW : 1;
-      else { p.w_first = first_slow ? SLOW : 1; p.w_last = last_slow ? SLOW : 1; }
-      // output depths whose depth taps reach outside x: all their stages take that path
-      const bool head_slow = g.p[0] > 0, tail_slow = g.out[0] - 1 - g.p[0] + g.k[0] > g.in[0];
-      if (g.out[0] == 1) p.wd_first = (head_slow || tail_slow) ? SLOW : 1;
-      else { p.wd_first = head_slow ? SLOW : 1; p.wd_last = tail_slow ? SLOW : 1; }
-    }
-  }
   // Every stage whole and every window inside x: the kernel without the border path (see ALLIN).
   const bool all_inside = even == 1 && xt == nullptr && g.p[0] == 0 && g.p[1] == 0 && g.p[2] == 0 &&
                           g.out[1] % SR == 0 && g.out[2] % SW == 0 && g.out[1] + 2 <= g.in[1] &&
                           g.out[2] + 2 <= g.in[2] && g.out[0] - 1 + g.k[0] <= g.in[0];
-  const int wgs = wg_count(p.total_stages);
   p.xt = static_cast<const uint16_t*>(xt);
   p.tlo_d = tlo ? tlo[0] : 0; p.tlo_h = tlo ? tlo[1] : 0; p.tlo_w = tlo ? tlo[2] : 0;
   p.tn_d = tn ? tn[0] : 0; p.tn_h = tn ? tn[1] : 0; p.tn_w = tn ? tn[2] : 0;
-  // One block of channels: g channels [gch, gch + cout_valid), x channels [xch, xch + cin_valid) of the
-  // tensors as they lie in memory (split mode: parts are channel groups), into out (+ gb_out).
-  auto run_block = [&](size_t gch, size_t xch, int cob, int cib, int cout_valid, int cin_valid, void* out,
-                       int out_cin_total, bool out32, bool accumulate, uint16_t* gb_out) -> int {
-    const int cgb = cob / 32, cxb = bl.KD * cib / 32;
-    p.Cin = cib; p.Cout = cob;
-    p.cin_valid = cin_valid; p.cout_valid = cout_valid;
-    p.x = static_cast<const uint16_t*>(x) + xch * x_cs;
-    p.g = static_cast<const uint16_t*>(go) + gch * g_cs;
-    p.bias_part = gb_out != nullptr ? p.part + (size_t)wgs * HALVES * 9 * cob * (bl.KD * cib) : nullptr;
-    int rc;
-    if (cgb == 2 && cxb == 2) rc = launch<2, 2>(p, even, f16, all_inside, wgs, s, who);
-    else if (cgb == 1 && cxb == 3) rc = launch<1, 3>(p, even, f16, all_inside, wgs, s, who);
-    else if (cgb == 1 && cxb == 1) rc = launch<1, 1>(p, even, f16, all_inside, wgs, s, who);
-    else if (cgb == 2 && cxb == 1) rc = launch<2, 1>(p, even, f16, all_inside, wgs, s, who);
-    else if (cgb == 1 && cxb == 2) rc = launch<1, 2>(p, even, f16, all_inside, wgs, s, who);
-    else JG_FAIL(JG_ERR_UNSUPPORTED, "%s: channel blocking (%d, %d) not built", who, cgb, cxb);
-    if (rc) return rc;
-    JG_CHECK_LAUNCH(who);
-    const int count = 9 * cob * bl.KD * cib;
-    if (out32)
-      wgrad_reduce_kernel<true><<<(count + 63) / 64, 256, 0, s>>>(out, p.part, wgs * HALVES, cob, bl.KD * cib, cib,
-                                                                    cout_valid, cin_valid, out_cin_total, accumulate);
-    else
-      wgrad_reduce_kernel<false><<<(count + 63) / 64, 256, 0, s>>>(out, p.part, wgs * HALVES, cob, bl.KD * cib, cib,
-                                                                     cout_valid, cin_valid, out_cin_total, 0);
-    JG_CHECK_LAUNCH(who);
-    if (gb_out != nullptr) {
-      wgrad_bias_reduce_kernel<<<(cob + 3) / 4, 256, 0, s>>>(gb_out, p.bias_part, wgs, cob, cout_valid);
-      JG_CHECK_LAUNCH(who);
-    }
-    return JG_OK;
-  };
+  JG_REQUIRE(plan.blocks() < 65536, "%s: too many channels", who);
+  const dim3 grid((unsigned)plan.wgs, (unsigned)plan.blocks());
+  int rc;
+  if (plan.cgb == 2 && plan.cxb == 2) rc = launch<2, 2>(p, even, f16, all_inside, grid, s, who);
+  else if (plan.cgb == 1 && plan.cxb == 3) rc = launch<1, 3>(p, even, f16, all_inside, grid, s, who);
+  else if (plan.cgb == 1 && plan.cxb == 1) rc = launch<1, 1>(p, even, f16, all_inside, grid, s, who);
+  else if (plan.cgb == 2 && plan.cxb == 1) rc = launch<2, 1>(p, even, f16, all_inside, grid, s, who);
+  else rc = launch<1, 2>(p, even, f16, all_inside, grid, s, who);
+  if (rc) return rc;
+  JG_CHECK_LAUNCH(who);
 
-  if (parts_fit_one_block(g, bl, parts)) {
-    // few channels: all part products in one launch (the parts are parts x cout and parts x cin
-    // channels of one block), then the ones that count are added up
-    const int cob = parts * g.cout > 32 ? 64 : 32, cib = parts * g.cin > 32 ? 64 : 32;  // within the block limits (checked)
-    int rc = run_block(0, 0, cob, cib, parts * g.cout, parts * g.cin, one_block_tmp, parts * g.cin, true, false, nullptr);
-    if (rc) return rc;
-    wgrad_combine_parts_kernel<<<(gw_count + 255) / 256, 256, 0, s>>>(sum32, one_block_tmp, g.cout, g.cin, bl.KD * 9,
-                                                                      parts);
+  ReduceParams r;
+  r.part = p.part; r.bias_part = p.bias_part;
+  r.gw = plan.parts_in_block > 1 ? one_block_tmp : gw;
+  r.gb = gb;
+  r.wgs = plan.wgs; r.npairs = plan.npairs;
+  r.pairs = plan.cgb * plan.cxb; r.GC = (int)plan.GC(); r.CXB = plan.cxb; r.cin_b = (int)plan.XC() / plan.KD;
+  r.KD = plan.KD; r.cin = p.cin; r.cout = p.cout; r.ci_blocks = plan.ci_blocks;
+  r.bias_cout = g.cout; r.bias_parts = parts;
+  r.gw_blocks = plan.co_blocks * plan.ci_blocks * 9 * r.pairs * 4;
+  const unsigned rgrid = (unsigned)r.gw_blocks + (gb != nullptr ? (unsigned)(g.cout + 63) / 64 : 0u);
+  if (dtype == JG_F32) wgrad_reduce_kernel<1><<<rgrid, 64 * RED_WAVES, 0, s>>>(r);
+  else if (f16) wgrad_reduce_kernel<2><<<rgrid, 64 * RED_WAVES, 0, s>>>(r);
+  else wgrad_reduce_kernel<0><<<rgrid, 64 * RED_WAVES, 0, s>>>(r);
+  JG_CHECK_LAUNCH(who);
+  if (plan.parts_in_block > 1) {
+    // few channels: all part products came from one block (the parts are channels of it); the ones that count
+    // are added up
+    const int gw_count = g.cout * g.cin * g.k[0] * 9;
+    wgrad_combine_parts_kernel<<<(gw_count + 255) / 256, 256, 0, s>>>(static_cast<float*>(gw), one_block_tmp, g.cout, g.cin,
+                                                                      plan.KD * 9, parts);
     JG_CHECK_LAUNCH(who);
-    return finish();
   }
-  for (int co0 = 0; co0 < g.cout;) {
-    const int cob = block_width(g.cout, co0, bl.cob);
-    for (int ci0 = 0; ci0 < g.cin;) {
-      const int cib = block_width(g.cin, ci0, bl.cib);
-      const int cin_valid = g.cin - ci0 < cib ? g.cin - ci0 : cib;
-      const int cout_valid = g.cout - co0 < cob ? g.cout - co0 : cob;
-      const size_t blk_at = ((size_t)co0 * g.cin + ci0) * bl.KD * 9;
-      for (int pr = 0; pr < npairs; ++pr) {
-        const int gpart = kPairs[first_pair + pr][0], xpart = kPairs[first_pair + pr][1];
-        void* out = (split || f16) ? static_cast<void*>(sum32 + blk_at)
-                                   : static_cast<void*>(static_cast<uint16_t*>(gw) + blk_at);
-        // the bias gradient comes from the g rows: once per block of output channels
-        uint16_t* gb_out = (gb != nullptr && ci0 == 0) ? static_cast<uint16_t*>(gb) + co0 : nullptr;
-        int rc = run_block((size_t)gpart * g.cout + co0, (size_t)xpart * g.cin + ci0, cob, cib, cout_valid, cin_valid,
-                           out, g.cin, split || f16, pr > 0, gb_out);
-        if (rc) return rc;
-      }
-      ci0 += cib;
-    }
-    co0 += cob;
-  }
-  return finish();
+  return JG_OK;
 }
 
 }  // namespace jg

@@ -170,6 +170,45 @@ def test_conv_primitives_match_oracle(case, dtype, dev):
     assert gb2.dtype == dtype and rel_l2(gb2, gb_want) < TOL[dtype], f"fused bias grad rel-L2 {rel_l2(gb2, gb_want):.3e}"
 
 
+# rows that start on odd pixels, windows over every edge, several blocks of channels a side with a short last one
+ODD_CASES = [
+    (2, 40, 72, (21, 131), (0, 0)),
+    (1, 70, 97, (9, 65), (2, 2)),
+    (1, 3, 5, (2, 3), (1, 1)),
+    (3, 17, 16, (16, 63), (0, 1)),
+    (1, 5, 33, (3, 5, 67), (1, 1, 1)),
+]
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", ODD_CASES, ids=lambda c: f"{c[1]}to{c[2]}_{'x'.join(map(str, c[3]))}_p{c[4][-1]}")
+def test_odd_rows_and_blocks_of_channels(case, dtype, offset, dev):
+    N, ci, co, size, pad = case
+    ns, ones = len(size), (1,) * len(size)
+    torch.manual_seed(11)
+
+    def placed(t):  # `offset` elements into its storage
+        flat = torch.empty(t.numel() + offset, dtype=dtype, device=dev)
+        flat[offset:] = t.to(dev).flatten()
+        return flat[offset:].view(t.shape)
+
+    x = torch.randn(N, ci, *size).to(dtype)
+    w = ((torch.rand(co, ci, *(3,) * ns) * 2 - 1) / (ci * 3**ns) ** 0.5).to(dtype)
+    b = torch.randn(co).to(dtype)
+    y_want = oc.forward(x.double(), w.double(), b.double(), ones, pad, ones)
+    g = torch.randn(y_want.shape).to(dtype)
+    xg, wg, gg = placed(x), w.to(dev), placed(g)
+    assert rel_l2(jc.conv_nd(xg, wg, b.to(dev), padding=pad), y_want) < TOL[dtype]
+    xd = x.double().requires_grad_(True)
+    wd = w.double().requires_grad_(True)
+    gx_want, gw_want = torch.autograd.grad(oc.forward(xd, wd, None, ones, pad, ones), (xd, wd), g.double())
+    assert rel_l2(jc.conv_nd_input(x.shape, wg, gg, padding=pad), gx_want) < TOL[dtype]
+    gw, gb = jc.conv_nd_weight(xg, w.shape, gg, padding=pad, with_bias_grad=True)
+    assert rel_l2(gw, gw_want) < TOL[dtype]
+    assert rel_l2(gb, g.double().sum(dim=(0, *range(2, 2 + ns)))) < TOL[dtype]
+
+
 def test_partial_channel_step_ignores_what_lies_behind_the_last_channel(dev):
     """3 input channels fill 3 of the 16 slots of an MFMA step; the slots behind them are read
     from whatever follows in memory (the next batch entry) and must not reach the result:
