@@ -924,7 +924,7 @@ __global__ __launch_bounds__(256) void fold_rows_kernel(Table tab,
           const uint32_t e = (uint32_t)ends(T(0), last_bits, strip_last, false, s_hi != nullptr);
           out.w = EB == 32 ? e : ((out.w & 0x0000ffffu) | (e << 16));
         }
-        *reinterpret_cast<u32x4_s4*>(drow + c0) = out;
+        store16_unaligned(drow + c0, out);
       }
     }
   }
@@ -1125,8 +1125,7 @@ extern "C" int jg_halo_assemble_3d(void* x_aug, const void* const src[27],
   const int Wa = g.lo[2] + g.n[2] + g.hi[2];
   RowPlan pl;
   const int V = 16 / elem_size;
-  if ((Wa * elem_size) % 4 == 0 &&
-      make_plan((unsigned long long)g.planes * Da * Ha, (Wa + V - 1) / V, Ha, Da, &pl)) {
+  if (make_plan((unsigned long long)g.planes * Da * Ha, (Wa + V - 1) / V, Ha, Da, &pl)) {
     const unsigned blocks = (unsigned)((((unsigned long long)pl.nrows << pl.lpr_log2) + 255) / 256);
     if (elem_size == 2)
       assemble_rows_kernel<uint16_t><<<blocks, 256, 0, s>>>(tab, static_cast<uint16_t*>(x_aug), g, pl);
@@ -1410,8 +1409,7 @@ extern "C" int jg_halo_fold_3d(void* gx, const void* gx_aug, const void* const s
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int V = 16 / es;
   RowPlan pl;
-  if ((g.n[2] * es) % 4 == 0 &&
-      make_plan((unsigned long long)g.planes * g.n[0] * g.n[1], (g.n[2] + V - 1) / V, g.n[1], g.n[0], &pl)) {
+  if (make_plan((unsigned long long)g.planes * g.n[0] * g.n[1], (g.n[2] + V - 1) / V, g.n[1], g.n[0], &pl)) {
     const unsigned blocks = (unsigned)((((unsigned long long)pl.nrows << pl.lpr_log2) + 255) / 256);
     // Two launches when the rows a D or H neighbour reaches are many enough to matter (more than one
     // row in 64) and fit the border kernel's indices: the row pass defers them, the border kernel
