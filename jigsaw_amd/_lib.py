@@ -17,6 +17,7 @@ import torch
 _LIB_PATH = Path(__file__).resolve().parent / "lib" / "libjigsaw_hip.so"
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
+_host = None
 
 JG_F32, JG_BF16, JG_F16 = 0, 1, 2
 _DTYPES = {torch.float32: JG_F32, torch.bfloat16: JG_BF16, torch.float16: JG_F16}
@@ -340,6 +341,19 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+def host():
+    """The native host module (``csrc/host.cpp``), imported once."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise LibraryMissing(f"jigsaw_amd/_host.so is not built or does not load ({e}). Run `python -m jigsaw_amd.build`.") from e
+        _host = module
+    return _host
+
+
 def abi_version() -> int:
     return int(load().jg_abi_version())
 
@@ -385,6 +399,11 @@ def stream_ptr(device: torch.device | None = None) -> c_void_p:
         index = device.index if device is not None and device.index is not None else torch.cuda.current_device()
         return c_void_p(_raw_stream(index))
     return c_void_p(torch.cuda.current_stream(device).cuda_stream)
+
+
+def stream_handle(device: torch.device) -> int:
+    """:func:`stream_ptr` as a plain number, for the native host module."""
+    return _raw_stream(device.index) if _raw_stream is not None else torch.cuda.current_stream(device).cuda_stream
 
 
 def i64_array(values) -> ctypes.Array:

@@ -1,8 +1,9 @@
-"""Build libjigsaw_hip.so (gfx950) from the HIP sources under ``csrc/``.
+"""Build libjigsaw_hip.so (gfx950) from the HIP sources under ``csrc/`` and, against it and
+torch, the native host module ``_host.so`` from ``csrc/host.cpp``.
 
 Usage: ``python -m jigsaw_amd.build [--jobs N] [--force]``. hipcc cross-compiles
 for gfx950 without a GPU present. Objects go to ``csrc/build/``, the library to
-``lib/libjigsaw_hip.so`` (both git-ignored; the library travels with the tree).
+``lib/libjigsaw_hip.so``, the module to ``_host.so`` (all git-ignored; the built files travel with the tree).
 """
 
 from __future__ import annotations
@@ -19,6 +20,7 @@ ROOT = Path(__file__).resolve().parent
 CSRC = ROOT / "csrc"
 OBJ = CSRC / "build"
 LIB = ROOT / "lib" / "libjigsaw_hip.so"
+HOST = ROOT / "_host.so"
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [
@@ -83,8 +85,41 @@ def _compile(src: Path, force: bool, extra: list[str]) -> Path:
     return obj
 
 
+def _run(cmd: list[str], what: str) -> None:
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"{what} failed:\n{proc.stderr}")
+
+
+def _compile_host(force: bool) -> Path:
+    """Object of ``csrc/host.cpp`` (no device code: the host compiler takes it)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    src, obj = CSRC / "host.cpp", OBJ / "host.o"
+    if not force and _newer(obj, [src, ROOT.parent / "include" / "jigsaw_hip.h"]):
+        return obj
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", "-DTORCH_EXTENSION_NAME=_host",
+           "-DTORCH_API_INCLUDE_EXTENSION_H", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    for path in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"]):
+        cmd += ["-isystem", path]
+    _run([*cmd, "-c", str(src), "-o", str(obj)], "g++ host.cpp")
+    return obj
+
+
+def _link_host(obj: Path) -> None:
+    from torch.utils import cpp_extension
+
+    cmd = ["g++", "-shared", "-o", str(HOST), str(obj), f"-L{LIB.parent}", "-ljigsaw_hip", "-Wl,-rpath,$ORIGIN/lib"]
+    for path in cpp_extension.library_paths():
+        cmd += [f"-L{path}", f"-Wl,-rpath,{path}"]
+    _run([*cmd, "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python"], "link of _host.so")
+
+
 def build(jobs: int = 8, force: bool = False, extra: list[str] | None = None) -> Path:
-    """Compile every ``csrc/*.hip`` and link ``lib/libjigsaw_hip.so``."""
+    """Compile every ``csrc/*.hip`` and link ``lib/libjigsaw_hip.so``; compile and link ``_host.so``."""
     extra = list(extra or [])
     OBJ.mkdir(parents=True, exist_ok=True)
     LIB.parent.mkdir(parents=True, exist_ok=True)
@@ -92,12 +127,15 @@ def build(jobs: int = 8, force: bool = False, extra: list[str] | None = None) ->
     if not srcs:
         raise RuntimeError(f"no HIP sources under {CSRC}")
     with cf.ThreadPoolExecutor(max_workers=max(1, jobs)) as pool:
+        host = pool.submit(_compile_host, force)
         objs = list(pool.map(lambda s: _compile(s, force, extra), srcs))
+        host_obj = host.result()
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(LIB)]
     cmd += [str(o) for o in objs]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stderr}")
+    _link_host(host_obj)
     return LIB
 
 

@@ -957,6 +957,43 @@ def _frame_decision(config, x, geom: HaloGeometry, weight_shape, kwargs):
     return frame_bands(x, geom, weight_shape, **kwargs)
 
 
+@lru_cache(maxsize=256)
+def _step(x_shape, dtype, w_shape, stride, padding, dilation, ranks, sizes, groups: int, fused_fold: bool):
+    """The native host plan (``csrc/host.cpp``) of a layer on a tile, or ``None`` where the Python route below runs it:
+    layers that are re-shaped before they reach the kernels, spans that the strips do not cover."""
+    n = len(w_shape) - 2
+    if dtype not in _lib._DTYPES or len(x_shape) != n + 2:
+        return None
+    if not spans_fit_the_strips(x_shape[-n:], w_shape[-n:], stride, padding, dilation, sizes):
+        return None
+    geom = HaloGeometry.for_conv(x_shape[-n:], w_shape[-n:], stride, padding, dilation, ranks, sizes)
+    lead, local_padding = tuple(x_shape[:2]), _local_padding(padding, sizes)
+    launches = [_launch_for(op, dtype, lead + geom.padded, w_shape, stride, local_padding, dilation, groups) for op in range(3)]
+    if any(launch is None for launch in launches):
+        return None
+    planes = lead[0] * lead[1]
+    present = set(_present_offsets(geom, ranks, sizes))
+    rows = {verb: [(o, i, lead + extent) for o, i, extent in rows] for verb, rows in geom._extents.items()}
+    sent = lambda verb: [row for row in rows[verb] if row[0] in present]  # noqa: E731
+    address = lambda c: ctypes.addressof(c)  # noqa: E731
+    return _lib.host().Step(
+        tuple(x_shape), lead + geom.padded, launches[0].shape, tuple(w_shape), dtype.itemsize, _lib.dtype_code(dtype),
+        address(geom.c_geom(planes)), address(geom.theirs().c_geom(planes)), geom.same_on_every_rank, address(launches[0].desc),
+        [launch.nbytes for launch in launches], rows["assemble"], rows["fold"], sent("pack_fwd"), sent("pack_bwd"),
+        fused_fold and dtype == torch.bfloat16 and groups == 1)
+
+
+def _step_for(config, x_shape, x, w, stride, padding, dilation, ranks, sizes):
+    if (not x.is_cuda or w.dtype != x.dtype or getattr(config, "framed", False) or config.conv_fn is not conv_nd
+            or config.conv_input_fn is not conv_nd_input or config.conv_weight_fn is not conv_nd_weight):
+        return None
+    try:
+        return _step(x_shape, x.dtype, w.shape, stride, padding, dilation, ranks, sizes, int(getattr(config, "groups_local", 1)),
+                     bool(getattr(config, "fused_fold", False)))
+    except TypeError:  # lists and the like do not hash
+        return None
+
+
 def conv_halo_nway(x, w, b, stride, padding, dilation, spatial_groups, channel_group, config):
     """Convolve with a halo exchange on every split axis; returns ``(y, x_aug)``.
 
@@ -974,6 +1011,14 @@ def conv_halo_nway(x, w, b, stride, padding, dilation, spatial_groups, channel_g
     n = config.n_spatial
     ranks, sizes = _mesh_position(spatial_groups)
     x = x.contiguous()
+    recv = None
+    step = _step_for(config, x.shape, x, w, stride, padding, dilation, ranks, sizes)
+    if step is not None:
+        stream = _lib.stream_handle(x.device)
+        recv = config.halo_exchange.forward(step.pack(x, stream)) if step.sends else {}
+        done = step.forward(x, recv, w, b, stream)
+        if done is not None:
+            return done
     kwargs = {"stride": stride, "padding": _local_padding(padding, sizes), "dilation": dilation, "groups": int(getattr(config, "groups_local", 1))}
     if not spans_fit_the_strips(x.shape[-n:], w.shape[-n:], stride, padding, dilation, sizes):
         # need spans that leave out owned rows or reach past the adjacent rank: one split axis at a
@@ -988,8 +1033,9 @@ def conv_halo_nway(x, w, b, stride, padding, dilation, spatial_groups, channel_g
         return y, x_aug
     geom = HaloGeometry.for_conv(x.shape[-n:], w.shape[-n:], stride, padding, dilation, ranks, sizes)
     present = _present_offsets(geom, ranks, sizes)
-    send = halo_pack(x, geom, from_padded=False, present=present) if present else {}
-    recv = config.halo_exchange.forward(send) if present else {}
+    if recv is None:
+        send = halo_pack(x, geom, from_padded=False, present=present) if present else {}
+        recv = config.halo_exchange.forward(send) if present else {}
     bands = _frame_decision(config, x, geom, w.shape, kwargs)
     if bands is not None:
         # only the frame of the padded tile is built; the kernels read the tile itself elsewhere.
@@ -1024,8 +1070,25 @@ def conv_halo_nway_backward(
     want_b = len(need) > 2
     need_b = want_b and need[2]
     g = grad_output.to(weight.dtype)
-    kwargs = {"stride": stride, "padding": local_padding, "dilation": dilation, "groups": int(getattr(config, "groups_local", 1))}
+    done = (lambda gx: (gx, g_w, g_b)) if want_b else (lambda gx: (gx, g_w))
     g_w = g_b = None
+    if x_tile is None and g.is_cuda and x_aug.dtype == g.dtype and not getattr(x_aug, "_jg_frame_only", False):
+        step = _step_for(config, (*x_aug.shape[:2], *local_in_spatial), x_aug, weight, stride, padding, dilation, ranks, sizes)
+        stream = _lib.stream_handle(g.device) if step is not None else 0
+        parts = step.backward(g, x_aug, weight, need_x, need_w, need_w and need_b, stream) if step is not None else None
+        if parts is not None:
+            part, g_w, g_b, send, folded = parts
+            if need_b and g_b is None:
+                g_b = config.grad_bias(g.contiguous())
+            if not need_x:
+                return done(None)
+            recv = config.halo_exchange.backward(send) if step.sends else {}
+            g_x = step.finish(part, folded, recv, stream)
+            if g_x is None:
+                geom = HaloGeometry.for_conv(local_in_spatial, weight.shape[-n:], stride, padding, dilation, ranks, sizes)
+                g_x = halo_fold_border_(part, recv, geom) if folded else halo_fold(part, recv, geom)
+            return done(g_x)
+    kwargs = {"stride": stride, "padding": local_padding, "dilation": dilation, "groups": int(getattr(config, "groups_local", 1))}
     if x_tile is None and need_w and getattr(config, "framed", False) and getattr(x_aug, "_jg_frame_only", False):
         raise RuntimeError(
             "x_aug is the frame of a framed forward (config.framed) and its interior is undefined: the weight "
@@ -1050,7 +1113,6 @@ def conv_halo_nway_backward(
     else:
         g_w = config.conv_weight_fn(x_aug, weight.shape, g, **kwargs) if need_w else None
         g_b = config.grad_bias(g.contiguous()) if need_b else None
-    done = (lambda gx: (gx, g_w, g_b)) if want_b else (lambda gx: (gx, g_w))
     if not need_x:
         return done(None)
     if not spans_fit_the_strips(local_in_spatial, weight.shape[-n:], stride, padding, dilation, sizes):
@@ -1231,9 +1293,9 @@ class _ConvNd(PositionalFunction):
         # the same decision conv_halo_nway took: x_aug is a frame only, so the tile is kept
         ctx.framed = False
         n = config.n_spatial
-        ranks, sizes = _mesh_position(spatial_groups)
         if (getattr(config, "framed", False) and isinstance(padding, tuple)
-                and spans_fit_the_strips(x.shape[-n:], weight.shape[-n:], stride, padding, dilation, sizes)):
+                and spans_fit_the_strips(x.shape[-n:], weight.shape[-n:], stride, padding, dilation, _mesh_position(spatial_groups)[1])):
+            ranks, sizes = _mesh_position(spatial_groups)
             geom = HaloGeometry.for_conv(x.shape[-n:], weight.shape[-n:], stride, padding, dilation, ranks, sizes)
             kwargs = {"stride": stride, "padding": _local_padding(padding, sizes), "dilation": dilation, "groups": int(getattr(config, "groups_local", 1))}
             x_c = x if x.dtype == x_aug.dtype else torch.empty(0, dtype=x_aug.dtype, device=x.device).new_empty(x.shape)
