@@ -204,10 +204,18 @@ def _embed_weight(w: torch.Tensor, off) -> torch.Tensor:
 # between its cells (backward). Costs prod(stride) times the matrix-core work of the strided
 # layer and a copy, and still beats the FMA kernels by an order of magnitude.
 # --------------------------------------------------------------------------- #
+def _strided_kernel(kernel, stride, dilation, padding) -> bool:
+    """3 x 3 at stride 2: the MFMA kernels take it as it is (all three passes)."""
+    return (tuple(kernel) == (3, 3) and tuple(stride) == (2, 2) and tuple(dilation) == (1, 1)
+            and padding is not None and all(p <= 2 for p in padding))
+
+
 def _dense_stride_ok(kernel, stride, dilation, padding=None) -> bool:
     if len(kernel) not in (2, 3) or all(s == 1 for s in stride):
         return False
     if all(k == s for k, s in zip(kernel, stride)):  # kernel = stride has its own route
+        return False
+    if _strided_kernel(kernel, stride, dilation, padding):
         return False
     ones = (1,) * len(kernel)
     if any(d != 1 for d in dilation):

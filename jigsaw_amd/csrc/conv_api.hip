@@ -170,7 +170,7 @@ extern "C" int jg_conv_fwd_framed(void* y, const void* x_frame, const void* x_ti
   int tlo[3], tn[3];
   rc = framed_extent(g, geom, "jg_conv_fwd_framed", tlo, tn);
   if (rc) return rc;
-  if (dtype != JG_BF16 || !jg::mfma_fwd_supported(g, dtype) || tn[2] % 2 != 0)
+  if (dtype != JG_BF16 || !jg::mfma_fwd_supported(g, dtype) || g.s[2] != 1 || tn[2] % 2 != 0)
     JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_fwd_framed: geometry / dtype has no framed kernel");
   return jg::mfma_fwd_framed(y, x_frame, x_tile, tlo, tn, w, bias, g, workspace, workspace_bytes,
                              static_cast<hipStream_t>(stream));

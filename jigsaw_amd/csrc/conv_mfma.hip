@@ -1,5 +1,5 @@
 // Implicit-GEMM convolution on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16):
-// 3x3 (2-D) and 3x3x3 (3-D), stride 1, dilation 1, channels-first tensors in and
+// 3x3 (2-D, stride 1 or 2) and 3x3x3 (3-D, stride 1), dilation 1, channels-first tensors in and
 // out. One kernel serves the forward pass and the input gradient.
 //
 //   GEMM view   Y[m][pixel] = sum_{tap, k} Wt[tap][m][k] * X[k][pixel + tap]
@@ -66,10 +66,10 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int KH = 3, KW = 3, TAPS = KH * KW;  // taps inside a plane
-constexpr int TH = 16, TW = 64;                // output tile of a workgroup
+constexpr int TILE_H = 16, TILE_W = 64;        // output tile of a workgroup (stride 2: half of it each way)
 constexpr int WAVES = 8, THREADS = WAVES * 64;
-constexpr int WROWS = 4;                       // output rows per wavefront
-constexpr int IN_ROWS = TH + KH - 1;           // 18
+constexpr int IN_ROWS = TILE_H + KH - 1;       // 18
+constexpr int IN_COLS = TILE_W + KW - 1;       // 66
 constexpr int OCTS = 9;                        // 9 octets of 8 pixels cover 66 (+6) columns
 constexpr int ROW_SLOTS = 8 * OCTS;            // 16-byte slots per LDS row
 constexpr int CK = 16;                         // contraction channels per stage
@@ -120,6 +120,8 @@ struct FwdParams {
   // x near the edges has to hold data. NULL: everything comes from x.
   const uint16_t* xt;
   int tlo_d, tlo_h, tlo_w, tn_d, tn_h, tn_w;
+  // MODE 2: extent of the produced tensor and the layer's padding; Hout, Wout count positions (i, j), pad_h = pad_w = 1
+  int Hx, Wx, px_h, px_w;
 };
 
 // Strips of the 26 neighbours, slot (dd+1)*9 + (dh+1)*3 + (dw+1); first kernel
@@ -142,29 +144,37 @@ __device__ __forceinline__ void* strip_entry(int idx) {
 // dst[(((mt*ngroups + group)*9 + tap9)*wc16 + c16 in group)*2 + kg][m_local][8 k] (bf16), contraction channel
 // k = kd*Cp + c (channels C..Cp-1 are zero padding). transposed = 0: A[m][k] = w[m][c][kd][kh][kw] (forward, w is
 // (M, C, KD, 3, 3)); transposed = 1: A[m][k] = w[c][m][KD-1-kd][2-kh][2-kw] (input
-// gradient, w is (C, M, KD, 3, 3)).
+// gradient, w is (C, M, KD, 3, 3)); transposed = 2: the six taps of a phase row of the strided input gradient
+// (see compute_phases), mt = 2 * channel tile + pa, w is (C, M, 3, 3).
+__device__ __forceinline__ bool phase_has(int pa, int tap) { return pa == 0 || tap >= 3; }
+__device__ __forceinline__ int phase_tap(int pa, int tap) {
+  const int kh = pa == 0 ? (tap < 3 ? 2 : 0) : 1, t = tap % 3;
+  return kh * KW + (t == 0 ? 2 : t == 1 ? 0 : 1);
+}
 __global__ __launch_bounds__(256) void prep_weights_kernel(uint16_t* __restrict__ dst,
                                                            const uint16_t* __restrict__ w,
                                                            int M, int C, int Cp, int KD, int MT, int mtiles,
                                                            int wc16, int ngroups, int transposed) {
   const int K = KD * Cp;
-  const int total = mtiles * ngroups * TAPS * wc16 * 2 * MT * 8;
+  const int taps = transposed == 2 ? 6 : TAPS;
+  const int total = mtiles * ngroups * taps * wc16 * 2 * MT * 8;
   for (int i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
     int e = i & 7;
     int r = i >> 3;
     int ml = r % MT; r /= MT;
     int kg = r & 1; r >>= 1;
     int c16l = r % wc16; r /= wc16;
-    int tap = r % TAPS; r /= TAPS;
+    int tap = r % taps; r /= taps;
     int grp = r % ngroups;
     int mt = r / ngroups;
-    const int m = mt * MT + ml;
+    const int m = (transposed == 2 ? mt >> 1 : mt) * MT + ml;
     const int k = (grp * wc16 + c16l) * CK + kg * 8 + e;
     uint16_t v = 0;  // rows past M and steps past K are padding
     const int kd = k / Cp, c = k - kd * Cp;
     if (m < M && k < K && c < C) {
       const int kh = tap / KW, kw = tap % KW;
-      if (!transposed)
+      if (transposed == 2) v = phase_has(mt & 1, tap) ? w[((size_t)c * M + m) * TAPS + phase_tap(mt & 1, tap)] : 0;
+      else if (!transposed)
         v = w[((((size_t)m * C + c) * KD + kd) * KH + kh) * KW + kw];
       else
         v = w[((((size_t)c * M + m) * KD + (KD - 1 - kd)) * KH + (KH - 1 - kh)) * KW + (KW - 1 - kw)];
@@ -232,24 +242,25 @@ __global__ __launch_bounds__(256) void prep_weights_split_kernel(uint16_t* __res
                                                                  int KD, int MT, int mtiles, int wc16, int ngroups,
                                                                  int transposed, int nblk, uint32_t wparts) {
   const int KB = KD * Cp, K = nblk * KB;
-  const int total = mtiles * ngroups * TAPS * wc16 * 2 * MT * 8;
+  const int taps = transposed == 2 ? 6 : TAPS;
+  const int total = mtiles * ngroups * taps * wc16 * 2 * MT * 8;
   for (int i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
     int e = i & 7;
     int r = i >> 3;
     int ml = r % MT; r /= MT;
     int kg = r & 1; r >>= 1;
     int c16l = r % wc16; r /= wc16;
-    int tap = r % TAPS; r /= TAPS;
+    int tap = r % taps; r /= taps;
     int grp = r % ngroups;
     int mt = r / ngroups;
-    const int m = mt * MT + ml;
+    const int m = (transposed == 2 ? mt >> 1 : mt) * MT + ml;
     const int k = (grp * wc16 + c16l) * CK + kg * 8 + e;
     const int blk = k / KB, kin = k - blk * KB;
     const int kd = kin / Cp, c = kin - kd * Cp;
     uint16_t v = 0;
-    if (m < M && k < K && c < C) {
+    if (m < M && k < K && c < C && (transposed != 2 || phase_has(mt & 1, tap))) {
       const int kh = tap / KW, kw = tap % KW;
-      const float f = to_float(!transposed ? w[((((size_t)m * C + c) * KD + kd) * KH + kh) * KW + kw]
+      const float f = to_float(transposed == 2 ? w[((size_t)c * M + m) * TAPS + phase_tap(mt & 1, tap)] : !transposed ? w[((((size_t)m * C + c) * KD + kd) * KH + kh) * KW + kw]
                                            : w[((((size_t)c * M + m) * KD + (KD - 1 - kd)) * KH + (KH - 1 - kh)) * KW + (KW - 1 - kw)]);
       v = split_part(f, (int)((wparts >> (2 * blk)) & 3u));
     }
@@ -281,6 +292,9 @@ __device__ inline void store_16_bytes(const void* base, uint32_t lane_off, u32x4
   // compiler pads that for its own stores but does not look inside an asm statement.
   asm volatile("global_store_dwordx4 %0, %1, %2\n\ts_nop 1" : : "v"(lane_off), "v"(v), "s"(base) : "memory");
 }
+__device__ inline void store_4_bytes(const void* base, uint32_t lane_off, uint32_t v) {
+  asm volatile("global_store_dword %0, %1, %2" : : "v"(lane_off), "v"(v), "s"(base) : "memory");
+}
 __device__ inline void store_f32(const void* base, uint32_t lane_off, float v) {
   asm volatile("global_store_dword %0, %1, %2" : : "v"(lane_off), "v"(v), "s"(base) : "memory");
 }
@@ -295,11 +309,28 @@ __device__ inline void store_f32(const void* base, uint32_t lane_off, float v) {
 // Used where every row segment of the result is made of whole, aligned 16-byte pieces.
 __device__ __forceinline__ int px_of_row(int m) { return (m & 0x13) | ((m & 4) << 1) | ((m & 8) >> 1); }
 
-template <int MT, bool EVEN, bool FOLD, bool FRAMED, bool F16 = false, bool PX = false>  // MT = produced channels per workgroup: 32 or 64
+// MODE 1: the forward pass at stride 2 along both axes. A tile is 8 x 32 produced pixels, whose window is the
+// same 18 x 72 pixels; the fragments of a tap take every second slot of a row, and with 64 produced channels a
+// wavefront owns 2 rows x 32 pixels of 32 channels.
+// MODE 2: the input gradient at stride 2. With ih + pad_h = 2 i + pa and iw + pad_w = 2 j + pb, a produced cell
+// sums the taps kh = pa + 2 a, kw = pb + 2 b over g[i - a][j - b]: each of the four phases (pa, pb) is a stride-1
+// convolution of g with 4, 2, 2 or 1 taps. A workgroup makes both pb of one pa (blockIdx.y = 2 * channel tile
+// + pa) for 16 x 64 positions (i, j) and 32 channels, so that a lane holds two neighbouring pixels of a row.
+// (The stride-1 kernels on every pixel, with a copy of every second one, took 66 + 16 us forward and 66 + 29 us
+// backward for 64 -> 128 channels of 4 x 257 x 257.)
+enum Mode { PLAIN = 0, STRIDED = 1, STRIDED_DGRAD = 2 };
+
+template <int MT, bool EVEN, bool FOLD, bool FRAMED, bool F16 = false, bool PX = false, int MODE = PLAIN>  // MT = produced channels per workgroup: 32 or 64
 __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips, FwdParams p) {
-  constexpr int CB = MT / 32;
+  static_assert(MODE == PLAIN || (!FOLD && !FRAMED), "strided layers have neither the fold epilogue nor the framed input");
+  static_assert(MODE != STRIDED_DGRAD || (MT == 32 && !PX), "32 channels of two phases");
+  constexpr int ST = MODE == STRIDED ? 2 : 1;
+  constexpr int TH = TILE_H / ST, TW = TILE_W / ST;
+  constexpr int WROWS = MODE != STRIDED ? 4 : MT / 32;                     // produced rows per wavefront
+  constexpr int CB = MODE == STRIDED ? 1 : MODE == STRIDED_DGRAD ? 2 : MT / 32;  // blocks of 32 channels (or phases) per wavefront
+  constexpr int WTAPS = MODE == STRIDED_DGRAD ? 6 : TAPS;                  // taps of prepared weights
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int w_slots = TAPS * p.wc16 * 2 * MT;  // 16-byte slots of one group of weights
+  const int w_slots = WTAPS * p.wc16 * 2 * MT;  // 16-byte slots of one group of weights
   u32x4* lds_w = reinterpret_cast<u32x4*>(smem);
   u32x4* lds_in = lds_w + w_slots;  // two stages
   float* lds_bias = reinterpret_cast<float*>(lds_in + 2 * STAGE_SLOTS);
@@ -310,8 +341,10 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   // Wavefronts w and w + 4 share a SIMD. They hold different column halves, so when a tile's second
   // half lies past the row end every SIMD drops half of that tile's MFMAs, and row groups two apart,
   // so a tile with few valid rows keeps two SIMDs busy instead of one.
-  const int wrow0 = ((wave + 2 * (wave >> 2)) & 3) * WROWS, wcol0 = (wave >> 2) * 32;
-  const int mt = blockIdx.y;
+  const int wrow0 = MODE != STRIDED ? ((wave + 2 * (wave >> 2)) & 3) * WROWS : (wave % (TH / WROWS)) * WROWS;
+  const int wcol0 = MODE != STRIDED ? (wave >> 2) * 32 : 0;
+  const int mt = MODE == STRIDED_DGRAD ? blockIdx.y >> 1 : blockIdx.y;
+  const int ch0 = MODE == STRIDED ? __builtin_amdgcn_readfirstlane(wave / (TH / WROWS)) * 32 : 0;  // the wavefront's first channel inside the tile
 
   // ---- tile schedule: XCD x (= blockIdx.x % 8) owns a contiguous range of tiles and
   // walks it cyclically from a start that differs per XCD. Without the stagger, ranges
@@ -338,7 +371,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   // workgroup; with more (many input channels) group g is loaded before the stages that
   // contract its channels.
   auto load_weights = [&](int grp) {
-    const u32x4* src = p.wprep + ((size_t)mt * p.ngroups + grp) * w_slots;
+    const u32x4* src = p.wprep + ((size_t)blockIdx.y * p.ngroups + grp) * w_slots;
     for (int i = tid; i < w_slots; i += THREADS) lds_w[i] = src[i];
   };
   if (p.ngroups == 1) load_weights(0);
@@ -409,14 +442,14 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     if (ti >= my_tiles) return;
     const TileCoord tc = coord(tile_of(ti));
     cur.od = tc.od;
-    cur.ih0 = tc.th * TH - p.pad_h;
-    cur.iw0 = tc.tw * TW + p.org_w - p.pad_w - p.lead;
-    cur.window_in = cur.ih0 >= 0 && cur.ih0 + IN_ROWS <= p.Hin && cur.iw0 >= 0 && cur.iw0 + p.lead + TW + KW - 1 <= p.Win;
+    cur.ih0 = ST * (tc.th * TH) - p.pad_h;
+    cur.iw0 = ST * (tc.tw * TW) + p.org_w - p.pad_w - p.lead;  // (org_w is 0 in the strided modes)
+    cur.window_in = cur.ih0 >= 0 && cur.ih0 + IN_ROWS <= p.Hin && cur.iw0 >= 0 && cur.iw0 + p.lead + IN_COLS <= p.Win;
     cur.base = reinterpret_cast<const char*>(p.x) +
                2 * ((ptrdiff_t)((size_t)tc.n * p.Cx * chan_stride) + (ptrdiff_t)cur.ih0 * p.Win + cur.iw0);
     if (FRAMED) {
       const int ht = cur.ih0 - p.tlo_h, wt = cur.iw0 - p.tlo_w;
-      cur.window_in_t = ht >= 0 && ht + IN_ROWS <= p.tn_h && wt >= 0 && wt + p.lead + TW + KW - 1 <= p.tn_w;
+      cur.window_in_t = ht >= 0 && ht + IN_ROWS <= p.tn_h && wt >= 0 && wt + p.lead + IN_COLS <= p.tn_w;
       cur.base_t = reinterpret_cast<const char*>(p.xt) +
                    2 * ((ptrdiff_t)((size_t)tc.n * p.Cx * chan_stride_t) + (ptrdiff_t)ht * p.tn_w + wt);
     }
@@ -615,7 +648,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   f32x16 acc[CB][WROWS];
 
   // One third (one kw) of a stage's MFMAs. The fragments roll through the stage: the weight
-  // fragments of tap row kh are last used by input row kh + WROWS - 1 of the group, and the
+  // fragments of tap row kh are last used by input row kh + ST * (WROWS - 1) of the group, and the
   // same registers are refilled right there with the next group's fragments (the next kw, or
   // after the last kw the first group of the next stage: the weights do not change at the
   // barrier), and the group's last step requests the first input fragment of the next kw. So
@@ -625,11 +658,11 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   int a_step = -1;  // the step inside the weight group whose kw = 0 fragments `a` holds
   auto weight_frag = [&](int wstep, int kh, int kw, int cb) {
     const u32x4* wt = lds_w + ((size_t)wstep * 2 + kg) * MT + ln;
-    return __builtin_bit_cast(bf16x8, wt[(size_t)(kh * KW + kw) * p.wc16 * 2 * MT + cb * 32]);
+    return __builtin_bit_cast(bf16x8, wt[(size_t)(kh * KW + kw) * p.wc16 * 2 * MT + ch0 + cb * 32]);
   };
   auto compute_kw = [&](int buf, int wstep, int kw, int wstep_next) {  // wstep: the stage's step inside its weight group
-    const u32x4* in = lds_in + buf * STAGE_SLOTS + kg * (IN_ROWS * ROW_SLOTS) + wrow0 * ROW_SLOTS;
-    const int col0 = wcol0 + (PX ? px_of_row(ln) : ln) + p.lead;  // the tile's pixel 0 sits `lead` slots into the staged row
+    const u32x4* in = lds_in + buf * STAGE_SLOTS + kg * (IN_ROWS * ROW_SLOTS) + ST * wrow0 * ROW_SLOTS;
+    const int col0 = wcol0 + ST * (PX ? px_of_row(ln) : ln) + p.lead;  // the tile's pixel 0 sits `lead` slots into the staged row
     const u32x4* inb = in + in_slot(col0 + kw);
     if (kw == 0) {
       if (a_step != wstep) {  // wave-uniform: the first stage, after a tile without work, after a weight reload
@@ -643,15 +676,15 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     // software pipeline over the input rows: the fragment of row rho+1 is requested
     // before the MFMAs of row rho are issued, so its LDS latency hides behind them
 #pragma unroll
-    for (int rho = 0; rho < WROWS + KH - 1; ++rho) {
+    for (int rho = 0; rho < ST * (WROWS - 1) + KH; ++rho) {
       const bf16x8 b = __builtin_bit_cast(bf16x8, bnext);
-      if (rho + 1 < WROWS + KH - 1) bnext = inb[(rho + 1) * ROW_SLOTS];
+      if (rho + 1 < ST * (WROWS - 1) + KH) bnext = inb[(rho + 1) * ROW_SLOTS];
       else if (kw + 1 < KW) bnext = in[in_slot(col0 + kw + 1)];
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int kh = 0; kh < KH; ++kh) {
-        const int r = rho - kh;
-        if (r >= 0 && r < WROWS) {
+        const int r = (rho - kh) / ST;
+        if (rho >= kh && (rho - kh) % ST == 0 && r < WROWS) {
 #pragma unroll
           for (int cb = 0; cb < CB; ++cb)
             if (F16 && PX)
@@ -667,7 +700,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
         }
       }
       __builtin_amdgcn_sched_barrier(0);
-      const int kh_done = rho - (WROWS - 1);  // this tap row's weights are not read again in this group
+      const int kh_done = rho - ST * (WROWS - 1);  // this tap row's weights are not read again in this group
       if (kh_done >= 0) {
         if (kw + 1 < KW) {
 #pragma unroll
@@ -682,13 +715,49 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     if (kw == KW - 1) a_step = p.ngroups == 1 ? wstep_next : -1;
   };
 
+  // MODE 2: the products of one column offset of g. Prepared taps: 3 kh' + t, row offset kh' (kh = 2, 0 of phase
+  // row 0 or none, 1 of phase row 1), t = 0: kw 2, read at column offset 0; 1: kw 0 and 2: kw 1, at offset 1. The
+  // accumulators are [pb][row].
+  auto compute_phases = [&](int buf, int wstep, int kw) __attribute__((always_inline)) {
+    const bool upper = (blockIdx.y & 1) == 0;  // pa = 0: both row offsets have taps
+    const u32x4* in = lds_in + buf * STAGE_SLOTS + kg * (IN_ROWS * ROW_SLOTS) + wrow0 * ROW_SLOTS + in_slot(wcol0 + ln + p.lead + kw);
+    const u32x4* wt = lds_w + ((size_t)wstep * 2 + kg) * MT + ln;
+    auto frag = [&](int tap) { return __builtin_bit_cast(bf16x8, wt[(size_t)tap * p.wc16 * 2 * MT]); };
+    auto mfma = [&](const bf16x8& w, const bf16x8& b, f32x16& to) __attribute__((always_inline)) {
+      to = F16 ? __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, b), to, 0, 0, 0)
+               : __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, b, to, 0, 0, 0);
+    };
+    bf16x8 w0[2], w1[2];
+    u32x4 next = in[0];
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh) {
+      w0[kh] = frag(3 * kh + (kw == 0 ? 0 : 1));
+      if (kw == 1) w1[kh] = frag(3 * kh + 2);
+    }
+#pragma unroll
+    for (int rho = 0; rho < WROWS + 1; ++rho) {
+      const bf16x8 b = __builtin_bit_cast(bf16x8, next);
+      if (rho < WROWS) next = in[(rho + 1) * ROW_SLOTS];
+      __builtin_amdgcn_sched_barrier(0);
+      if (rho < WROWS && upper) {
+        mfma(w0[0], b, acc[0][rho]);
+        if (kw == 1) mfma(w1[0], b, acc[CB - 1][rho]);
+      }
+      if (rho > 0) {
+        mfma(w0[1], b, acc[0][rho - 1]);
+        if (kw == 1) mfma(w1[1], b, acc[CB - 1][rho - 1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
   // Accumulator lane (ln, kg), register i of block cb: produced channel
   // cb*32 + 8*(i/4) + 4*kg + i%4, pixel column wcol0 + ln.
   auto init_acc = [&]() {
     if (PX) {  // a lane owns one channel per block
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb) {
-        const float bv = lds_bias[cb * 32 + ln];
+        const float bv = lds_bias[ch0 + cb * 32 + ln];
 #pragma unroll
         for (int r = 0; r < WROWS; ++r)
 #pragma unroll
@@ -700,7 +769,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const f32x4 bv = *reinterpret_cast<const f32x4*>(lds_bias + cb * 32 + 8 * j + 4 * kg);
+        const f32x4 bv = *reinterpret_cast<const f32x4*>(lds_bias + ch0 + (MODE == STRIDED_DGRAD ? 0 : cb * 32) + 8 * j + 4 * kg);
 #pragma unroll
         for (int r = 0; r < WROWS; ++r) {
           acc[cb][r][4 * j + 0] = bv.x;
@@ -743,11 +812,11 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     const int m_lane = (l4 & 8) + ((l4 >> 1) & 3) + ((l4 & 1) << 2);
     const uint32_t voff = (uint32_t)(m_lane * chan_bytes) + 16u * (lane & 3) + row_off;
     // all the row's pieces are requested before the first is stored: one LDS latency per row
-    u32x4 piece[MT / 16];
+    u32x4 piece[2 * CB];
 #pragma unroll
-    for (int q = 0; q < MT / 16; ++q) piece[q] = *reinterpret_cast<const u32x4*>(scratch + (q * 64 + lane) * 16);
+    for (int q = 0; q < 2 * CB; ++q) piece[q] = *reinterpret_cast<const u32x4*>(scratch + (q * 64 + lane) * 16);
 #pragma unroll
-    for (int q = 0; q < MT / 16; ++q) store_16_bytes(ytile + (size_t)q * 16 * chan_bytes, voff, piece[q]);
+    for (int q = 0; q < 2 * CB; ++q) store_16_bytes(ytile + (size_t)q * 16 * chan_bytes, voff, piece[q]);
   };
 
   // PX layout: lane (ln, kg) holds channel cb * 32 + ln; registers 8 J .. 8 J + 7 hold the pixels
@@ -775,8 +844,8 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     // wave-uniform base: the tile's first column in produced channel mt * MT, row 0 (it may lie before
     // the row where the tile grid starts left of the tensor; such pieces are not stored)
     char* ytile = reinterpret_cast<char*>(p.y) +
-                  2 * ((ptrdiff_t)(((size_t)tc.n * p.M + (size_t)mt * MT) * ochan + (size_t)tc.od * plane_o) + (ptrdiff_t)tw0);
-    const int m_left = p.M - mt * MT;
+                  2 * ((ptrdiff_t)(((size_t)tc.n * p.M + (size_t)mt * MT + ch0) * ochan + (size_t)tc.od * plane_o) + (ptrdiff_t)tw0);
+    const int m_left = p.M - mt * MT - ch0;
     const int l4 = lane >> 2, pc = lane & 3;  // reading side: channel 16 q + l4, piece pc
     const int px = tw0 + wcol0 + 8 * pc;
     const bool px_ok = px >= 0 && px + 8 <= p.Wout;
@@ -792,13 +861,13 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
 #pragma unroll
         for (int J = 0; J < 2; ++J)
           *reinterpret_cast<u32x4*>(wr + cb * 32 * 64 + (((2 * J + kg) ^ wsw) << 4)) = piece_16bit(cb, r, J);
-      u32x4 piece[MT / 16];
+      u32x4 piece[2 * CB];
 #pragma unroll
-      for (int q = 0; q < MT / 16; ++q) piece[q] = *reinterpret_cast<const u32x4*>(rd + q * 16 * 64);
+      for (int q = 0; q < 2 * CB; ++q) piece[q] = *reinterpret_cast<const u32x4*>(rd + q * 16 * 64);
       if (oh < p.Hout) {
         const uint32_t row_off = lane_off + 2u * (uint32_t)oh * (uint32_t)p.Wout;
 #pragma unroll
-        for (int q = 0; q < MT / 16; ++q)
+        for (int q = 0; q < 2 * CB; ++q)
           if (px_ok && q * 16 + l4 < m_left) store_16_bytes(ytile + (size_t)q * 16 * chan_bytes, row_off, piece[q]);
       }
     }
@@ -812,7 +881,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
         tw0 + wcol0 >= 0 && tw0 + wcol0 + 32 <= p.Wout) {  // wave-uniform
       unsigned char* scratch = reinterpret_cast<unsigned char*>(lds_in + free_buf * STAGE_SLOTS) + wave * (STAGE_BYTES / WAVES);
       char* ytile = reinterpret_cast<char*>(p.y) +
-                    2 * (((size_t)tc.n * p.M + (size_t)mt * MT) * (plane_o * p.Dout) + (size_t)tc.od * plane_o +
+                    2 * (((size_t)tc.n * p.M + (size_t)mt * MT + ch0) * (plane_o * p.Dout) + (size_t)tc.od * plane_o +
                          (size_t)tw0);
 #pragma unroll
       for (int r = 0; r < WROWS; ++r) {
@@ -828,11 +897,11 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
       return;
     }
     char* ybase = reinterpret_cast<char*>(p.y) +
-                  2 * (((size_t)tc.n * p.M + (size_t)mt * MT) * ochan + (size_t)tc.od * plane_o);
-    const int m_left = p.M - mt * MT - 4 * kg;  // channels from this lane's first one to the end
+                  2 * (((size_t)tc.n * p.M + (size_t)mt * MT + ch0) * ochan + (size_t)tc.od * plane_o);
+    const int m_left = p.M - mt * MT - ch0 - 4 * kg;  // channels from this lane's first one to the end
     if (p.out_kind == 1) {  // uniform: the same walk with 4-byte stores
       char* ybase32 = reinterpret_cast<char*>(p.y) +
-                      4 * (((size_t)tc.n * p.M + (size_t)mt * MT) * ochan + (size_t)tc.od * plane_o);
+                      4 * (((size_t)tc.n * p.M + (size_t)mt * MT + ch0) * ochan + (size_t)tc.od * plane_o);
 #pragma unroll
       for (int r = 0; r < WROWS; ++r) {
         const int oh = tc.th * TH + wrow0 + r;
@@ -877,8 +946,49 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
       }
     }
   };
+  // MODE 2: a lane's two phases are neighbouring pixels of a row and leave together, at whatever alignment the
+  // row has (4-byte stores at 2-byte aligned addresses run at the rate of aligned ones).
+  auto epilogue_phases = [&](const TileCoord& tc) {
+    const int pa = blockIdx.y & 1;
+    const int iw = 2 * (tc.tw * TW + wcol0 + ln) - p.px_w;
+    const bool ok0 = iw >= 0 && iw < p.Wx, ok1 = iw + 1 >= 0 && iw + 1 < p.Wx;
+    const size_t plane_x = (size_t)p.Hx * p.Wx;
+    const int m_left = p.M - mt * MT - 4 * kg;
+    // a wave-uniform base and a 32-bit lane offset that walks the channels by additions
+    const uint32_t es = p.out_kind == 1 ? 4u : 2u;
+    const char* const base = reinterpret_cast<const char*>(p.y) + es * (((size_t)tc.n * p.M + (size_t)mt * MT) * plane_x);
+    const uint32_t st = es * (uint32_t)plane_x;
+#pragma unroll
+    for (int r = 0; r < WROWS; ++r) {
+      const int ih = 2 * (tc.th * TH + wrow0 + r) + pa - p.px_h;
+      if (ih < 0 || ih >= p.Hx) continue;
+      const uint32_t row = 4 * kg * st + es * (uint32_t)(ih * p.Wx + iw);
+      auto walk = [&](auto store) __attribute__((always_inline)) {
+        uint32_t vo = row;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          if (8 * (i >> 2) + (i & 3) < m_left) store(i, vo);
+          vo += (i & 3) == 3 ? 5 * st : st;
+        }
+      };
+      if (p.out_kind == 1) {
+        if (ok0) walk([&](int i, uint32_t vo) { store_f32(base, vo, acc[0][r][i]); });
+        if (ok1) walk([&](int i, uint32_t vo) { store_f32(base, vo + 4, acc[CB - 1][r][i]); });
+        continue;
+      }
+      auto pair = [&](int i) {
+        f32x2 v2 = {acc[0][r][i], acc[CB - 1][r][i]};
+        return F16 ? __builtin_bit_cast(uint32_t, __builtin_convertvector(v2, f16x2))
+                   : __builtin_bit_cast(uint32_t, __builtin_convertvector(v2, bf16x2));
+      };
+      if (ok0 && ok1) walk([&](int i, uint32_t vo) { store_4_bytes(base, vo, pair(i)); });
+      else if (ok0) walk([&](int i, uint32_t vo) { store_bf16_lo(base, vo, pair(i)); });
+      else if (ok1) walk([&](int i, uint32_t vo) { store_bf16_hi(base, vo + 2, pair(i)); });
+    }
+  };
   auto epilogue = [&](const TileCoord& tc, int free_buf) {
-    if (PX) epilogue_px(tc, free_buf);
+    if constexpr (MODE == STRIDED_DGRAD) epilogue_phases(tc);
+    else if (PX) epilogue_px(tc, free_buf);
     else if ((mt + 1) * MT <= p.M) epilogue_rows(tc, std::false_type{}, free_buf);
     else epilogue_rows(tc, std::true_type{}, free_buf);
   };
@@ -1024,7 +1134,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   // through LDS to leave as 16-byte pieces), and the fold's does where the tile grid lies on the 16-byte grid
   // of the unpadded gradient (the same test as in epilogue_fold; it is the same for every tile of a launch).
   const bool epilogue_uses_lds =
-      !FOLD || ((((p.org_w - p.lo_w) & 7) == 0) && (p.nW & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
+      MODE == STRIDED_DGRAD ? false : !FOLD || ((((p.org_w - p.lo_w) & 7) == 0) && (p.nW & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
   int buf = 0;
   cursor_enter(0);
   issue_stage();
@@ -1058,8 +1168,12 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
         if (q + 2 < stages) issue_stage();
       }
       if (live) {
-        compute_kw(buf, wstep, 0, wstep_next);
-        compute_kw(buf, wstep, 1, wstep_next);
+        if constexpr (MODE == STRIDED_DGRAD) {
+          compute_phases(buf, wstep, 0);
+        } else {
+          compute_kw(buf, wstep, 0, wstep_next);
+          compute_kw(buf, wstep, 1, wstep_next);
+        }
       }
       // the buffer written next was the last epilogue's scratch (the fold's 2-byte stores leave from the registers:
       // nothing to wait for, and the wavefronts that are through with their stores do not wait for the others here)
@@ -1068,7 +1182,13 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
         if (q + 1 < stages) store_stage(buf ^ 1, q + 1);  // other buffer: no hazard with this stage's reads
         if (q + 2 < stages) issue_stage();
       }
-      if (live) compute_kw(buf, wstep, 2, wstep_next);
+      if (live) {
+        if constexpr (MODE == STRIDED_DGRAD) {
+          compute_phases(buf, wstep, 1);
+        } else {
+          compute_kw(buf, wstep, 2, wstep_next);
+        }
+      }
       __syncthreads();
       buf ^= 1;
       if (++wstep == p.wc16) {
@@ -1107,20 +1227,22 @@ struct Layout {
 
 int pad16(int c) { return (c + CK - 1) / CK * CK; }
 
-// K: contraction length with the channels padded to a multiple of 16 per depth tap
-Layout layout_of(int K, int M) {
+// K: contraction length with the channels padded to a multiple of 16 per depth tap. phases: the strided
+// input gradient, tiles of 32 channels twice (one for each phase row), six taps each.
+Layout layout_of(int K, int M, bool phases = false) {
   Layout L;
+  const int taps = phases ? 6 : TAPS;
   const int mpad = (M + 31) / 32 * 32;
-  L.MT = (mpad % 64 == 0) ? 64 : 32;
-  L.mtiles = mpad / L.MT;
+  L.MT = (mpad % 64 == 0 && !phases) ? 64 : 32;
+  L.mtiles = mpad / L.MT * (phases ? 2 : 1);
   L.nc16 = K / CK;
   const size_t budget = 160 * 1024 - 2 * (size_t)STAGE_BYTES - L.MT * 4;
-  int cap = (int)(budget / ((size_t)TAPS * 2 * L.MT * 16));
+  int cap = (int)(budget / ((size_t)taps * 2 * L.MT * 16));
   if (cap < 1) cap = 1;
   L.wc16 = L.nc16 < cap ? L.nc16 : cap;
   if (L.wc16 < 1) L.wc16 = 1;
   L.ngroups = (L.nc16 + L.wc16 - 1) / L.wc16;
-  const size_t slots = (size_t)TAPS * L.wc16 * 2 * L.MT;
+  const size_t slots = (size_t)taps * L.wc16 * 2 * L.MT;
   L.prep_bytes = (size_t)L.mtiles * L.ngroups * slots * 16;
   L.lds_bytes = slots * 16 + 2 * (size_t)STAGE_BYTES + L.MT * 4;
   return L;
@@ -1131,8 +1253,9 @@ bool shape_ok(int C, int M, const ConvGeom& g) {
   if (g.k[1] != KH || g.k[2] != KW) return false;
   if (g.k[0] != 1 && g.k[0] != 3) return false;
   if (g.k[0] == 1 && (g.in[0] != 1 || g.p[0] != 0)) return false;
+  const bool strided = g.s[1] == 2 && g.s[2] == 2 && g.k[0] == 1;
   for (int a = 0; a < 3; ++a)
-    if (g.s[a] != 1 || g.d[a] != 1) return false;
+    if ((g.s[a] != 1 && !(strided && a > 0)) || g.d[a] != 1) return false;
   if (C <= 0 || M <= 0) return false;
   // per-lane byte offsets inside one batch entry are 32-bit
   const size_t in_sz = (size_t)g.in[0] * g.in[1] * g.in[2], out_sz = (size_t)g.out[0] * g.out[1] * g.out[2];
@@ -1140,7 +1263,6 @@ bool shape_ok(int C, int M, const ConvGeom& g) {
   return big * 2 * 72 < (1ull << 31);
 }
 
-size_t prep_bytes(int K, int M) { return layout_of(K, M).prep_bytes; }
 
 struct Launch {
   const void* x;
@@ -1152,6 +1274,8 @@ struct Launch {
   int N, C, M, KD;
   int Din, Hin, Win, Dout, Hout, Wout;
   int pad_d, pad_h, pad_w;
+  int mode;                 // Mode of the kernel
+  int px_h, px_w;           // STRIDED_DGRAD: the layer's padding
   int transposed;
   int fold;                 // fold mode: y is the unpadded tile, strips receive the halo cells
   int lo[3], n[3];          // own extent inside the produced tensor (fold mode)
@@ -1162,9 +1286,9 @@ struct Launch {
 
 // Bytes of the split copy of an input (its bf16 parts), rounded to 256
 size_t split_bytes(size_t elements, int parts) { return (elements * parts * 2 + 255) / 256 * 256; }
-size_t conv_ws_bytes(int split, int KD, int C, int M, size_t x_elements) {
+size_t conv_ws_bytes(int split, int KD, int C, int M, size_t x_elements, bool phases) {
   const SplitSpec sp = split_spec(split);
-  const size_t prep = prep_bytes(sp.nblk * KD * pad16(C), M);
+  const size_t prep = layout_of(sp.nblk * KD * pad16(C), M, phases).prep_bytes;
   return split ? (prep + 255) / 256 * 256 + split_bytes(x_elements, sp.parts) : prep;
 }
 
@@ -1184,12 +1308,13 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
   const int nblk = sp.nblk;
   const int K = nblk * L.KD * pad16(L.C);
   const size_t x_elements = (size_t)L.N * L.C * L.Din * L.Hin * L.Win;
-  const size_t need = conv_ws_bytes(L.split, L.KD, L.C, L.M, x_elements);
+  const bool phases = L.mode == STRIDED_DGRAD;
+  const size_t need = conv_ws_bytes(L.split, L.KD, L.C, L.M, x_elements, phases);
   if (ws == nullptr || ws_bytes < need)
     JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, ws_bytes, need);
   JG_REQUIRE((reinterpret_cast<uintptr_t>(ws) & 15) == 0, "%s: workspace must be 16-byte aligned",
              who);
-  const Layout lay = layout_of(K, L.M);
+  const Layout lay = layout_of(K, L.M, phases);
   const int MT = lay.MT;
   uint16_t* wprep = static_cast<uint16_t*>(ws);
   const size_t total_w = lay.prep_bytes / 2;
@@ -1230,22 +1355,30 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
   p.Din = L.Din; p.Hin = L.Hin; p.Win = L.Win;
   p.Dout = L.Dout; p.Hout = L.Hout; p.Wout = L.Wout;
   p.pad_d = L.pad_d; p.pad_h = L.pad_h; p.pad_w = L.pad_w;
-  p.tiles_h = (L.Hout + TH - 1) / TH;
+  p.Hx = p.Wx = p.px_h = p.px_w = 0;
+  if (phases) {  // the kernel's grid runs over the positions (i, j)
+    p.Hx = L.Hout; p.Wx = L.Wout;
+    p.px_h = L.px_h; p.px_w = L.px_w;
+    p.Hout = (L.Hout - 1 + L.px_h) / 2 + 1;
+    p.Wout = (L.Wout - 1 + L.px_w) / 2 + 1;
+  }
+  const int TH = L.mode == STRIDED ? TILE_H / 2 : TILE_H, TW = L.mode == STRIDED ? TILE_W / 2 : TILE_W;
+  p.tiles_h = (p.Hout + TH - 1) / TH;
   // Where to put the tile grid. A tile's staged rows start at input column org_w + TW * tw - pad_w.
   // When the rows of x are a multiple of 128 bytes apart, an origin that makes this a multiple of
   // TW puts every staged row segment on a cache-line boundary (144 bytes: two lines instead of
   // three); it is taken when it costs no extra tile column.
   p.org_w = 0;
   // (not where it would take the 16-byte store path away: a plain 16-bit result with rows of whole pieces)
-  const bool wide_rows = !L.fold && L.split != 1 && L.Wout % 8 == 0;
-  if (!wide_rows && L.pad_w % TW != 0 && L.Win % 64 == 0 && (reinterpret_cast<uintptr_t>(x16) & 127) == 0) {
+  const bool wide_rows = !L.fold && L.split != 1 && L.Wout % 8 == 0 && !phases;
+  if (!wide_rows && L.mode == PLAIN && L.pad_w % TW != 0 && L.Win % 64 == 0 && (reinterpret_cast<uintptr_t>(x16) & 127) == 0) {
     const int org = L.pad_w % TW - TW;
     if ((L.Wout - org + TW - 1) / TW <= (L.Wout + TW - 1) / TW) p.org_w = org;
   }
   // rows of the staged windows start at even columns where `lead` can see to it: 4-byte aligned loads
   const bool even = (L.Win % 2 == 0) && ((reinterpret_cast<uintptr_t>(x16) & 3) == 0);
   p.lead = even ? (L.pad_w - p.org_w) & 1 : 0;
-  p.tiles_w = (L.Wout - p.org_w + TW - 1) / TW;
+  p.tiles_w = (p.Wout - p.org_w + TW - 1) / TW;
   p.sw = p.tiles_w;
   const long long tiles = (long long)L.N * L.Dout * p.tiles_h * p.tiles_w;
   JG_REQUIRE(tiles < (1ll << 30), "%s: too many tiles", who);
@@ -1270,7 +1403,24 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
   void (*kern)(StripTable, FwdParams) = nullptr;
   if (L.f16 && (L.fold || L.xt != nullptr))
     JG_FAIL(JG_ERR_UNSUPPORTED, "%s: the fold epilogue and the framed input are built for bf16 only", who);
-  if (L.fold) {
+  if (L.mode != PLAIN) {
+    const bool wide = wide_rows && (reinterpret_cast<uintptr_t>(L.y) & 15) == 0;
+    auto strided = [&](auto f16, auto px) {
+      constexpr bool F = decltype(f16)::value, X = decltype(px)::value;
+      if (MT == 64) kern = even ? &conv3x3_mfma_kernel<64, true, false, false, F, X, STRIDED> : &conv3x3_mfma_kernel<64, false, false, false, F, X, STRIDED>;
+      else kern = even ? &conv3x3_mfma_kernel<32, true, false, false, F, X, STRIDED> : &conv3x3_mfma_kernel<32, false, false, false, F, X, STRIDED>;
+    };
+    if (phases) {
+      if (L.f16) kern = even ? &conv3x3_mfma_kernel<32, true, false, false, true, false, STRIDED_DGRAD> : &conv3x3_mfma_kernel<32, false, false, false, true, false, STRIDED_DGRAD>;
+      else kern = even ? &conv3x3_mfma_kernel<32, true, false, false, false, false, STRIDED_DGRAD> : &conv3x3_mfma_kernel<32, false, false, false, false, false, STRIDED_DGRAD>;
+    } else if (L.f16) {
+      if (wide) strided(std::true_type{}, std::true_type{});
+      else strided(std::true_type{}, std::false_type{});
+    } else {
+      if (wide) strided(std::false_type{}, std::true_type{});
+      else strided(std::false_type{}, std::false_type{});
+    }
+  } else if (L.fold) {
     if (MT == 64) kern = even ? &conv3x3_mfma_kernel<64, true, true, false> : &conv3x3_mfma_kernel<64, false, true, false>;
     else kern = even ? &conv3x3_mfma_kernel<32, true, true, false> : &conv3x3_mfma_kernel<32, false, true, false>;
   } else if (L.xt != nullptr) {
@@ -1334,14 +1484,14 @@ bool mfma_dgrad_supported(const ConvGeom& g, int dtype) {
   if (!dtype_ok(g, dtype) || g.batch <= 0) return false;
   for (int a = 0; a < 3; ++a)
     if (g.p[a] > g.k[a] - 1) return false;
-  return shape_ok(g.cout, g.cin, g);
+  return shape_ok(g.cout, g.cin, g);  // (strides 1 and 2)
 }
 
 size_t mfma_fwd_workspace(const ConvGeom& g, int dtype) {
-  return conv_ws_bytes(split_mode(dtype), g.k[0], g.cin, g.cout, (size_t)g.batch * g.cin * g.in[0] * g.in[1] * g.in[2]);
+  return conv_ws_bytes(split_mode(dtype), g.k[0], g.cin, g.cout, (size_t)g.batch * g.cin * g.in[0] * g.in[1] * g.in[2], false);
 }
 size_t mfma_dgrad_workspace(const ConvGeom& g, int dtype) {
-  return conv_ws_bytes(split_mode(dtype), g.k[0], g.cout, g.cin, (size_t)g.batch * g.cout * g.out[0] * g.out[1] * g.out[2]);
+  return conv_ws_bytes(split_mode(dtype), g.k[0], g.cout, g.cin, (size_t)g.batch * g.cout * g.out[0] * g.out[1] * g.out[2], g.s[2] == 2);
 }
 
 static int fwd_launch(void* y, const void* x, const void* xt, const int* tlo, const int* tn, const void* w,
@@ -1355,6 +1505,8 @@ static int fwd_launch(void* y, const void* x, const void* xt, const int* tlo, co
   L.Din = g.in[0]; L.Hin = g.in[1]; L.Win = g.in[2];
   L.Dout = g.out[0]; L.Hout = g.out[1]; L.Wout = g.out[2];
   L.pad_d = g.p[0]; L.pad_h = g.p[1]; L.pad_w = g.p[2];
+  L.mode = g.s[2] == 2 ? STRIDED : PLAIN;
+  L.px_h = L.px_w = 0;
   L.transposed = 0;
   L.fold = 0;
   L.strips = nullptr;
@@ -1384,9 +1536,9 @@ void mfma_frame_bands(const ConvGeom& g, const int tlo[3], const int tn[3], int 
   // depth: a stage reads one plane; planes outside the tile are read whole
   band_lo[0] = tlo[0];
   band_hi[0] = g.in[0] - tlo[0] - tn[0];
-  const int tile[3] = {1, TH, TW};
+  const int tile[3] = {1, TILE_H, TILE_W};
   const int reach[3] = {1, IN_ROWS, OCTS * 8};  // cells a window may touch (the last octet in full)
-  const int need[3] = {1, IN_ROWS, TW + KW - 1};
+  const int need[3] = {1, IN_ROWS, IN_COLS};
   for (int a = 1; a < 3; ++a) {
     const int ntiles = (g.out[a] + tile[a] - 1) / tile[a];
     int first_in = -1, last_in = -1;  // tiles whose window lies inside [tlo, tlo + tn)
@@ -1426,7 +1578,14 @@ static int dgrad_launch(void* gx, void* const* strips, const int* lo, const int*
   L.Din = g.out[0]; L.Hin = g.out[1]; L.Win = g.out[2];
   L.Dout = g.in[0]; L.Hout = g.in[1]; L.Wout = g.in[2];
   L.pad_d = g.k[0] - 1 - g.p[0]; L.pad_h = KH - 1 - g.p[1]; L.pad_w = KW - 1 - g.p[2];
+  L.mode = PLAIN;
+  L.px_h = g.p[1]; L.px_w = g.p[2];
   L.transposed = 1;
+  if (g.s[2] == 2) {
+    L.mode = STRIDED_DGRAD;
+    L.transposed = 2;
+    L.pad_h = L.pad_w = 1;
+  }
   L.fold = lo != nullptr;
   L.strips = strips;
   L.xt = nullptr;
@@ -1445,6 +1604,7 @@ int mfma_dgrad(void* gx, const void* w, const void* go, const ConvGeom& g, void*
 
 int mfma_dgrad_fold(void* gx, void* const strips[27], const int lo[3], const int n[3], const void* w,
                     const void* go, const ConvGeom& g, void* ws, size_t ws_bytes, hipStream_t s) {
+  if (g.s[2] != 1) JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_dgrad_fold(mfma): strided layers only have the unfused path");
   // the fold epilogue has no path for a ragged last tile of produced channels
   const Layout lay = layout_of(g.k[0] * pad16(g.cout), g.cin);
   if (lay.mtiles * lay.MT != g.cin)

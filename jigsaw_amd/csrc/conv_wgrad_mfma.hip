@@ -1,5 +1,5 @@
 // Weight gradient of the 3x3 (2-D) and 3x3x3 (3-D) convolution on the bf16 matrix
-// cores, stride 1, dilation 1, channels-first tensors; a workgroup covers a block of 32 or
+// cores, stride 1 (2-D also stride 2), dilation 1, channels-first tensors; a workgroup covers a block of 32 or
 // 64 channels a side, any other channel counts are more blocks of the same launch. Optionally the
 // bias gradient from the same pass over g. fp16 tensors run the same kernel on the fp16
 // MFMA instruction (the gradient is reduced in fp32 and rounded to fp16 once); fp32 tensors
@@ -54,13 +54,24 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
-constexpr int SR = 2, SW = 64;        // output rows / columns per stage
-constexpr int XR = SR + 2;            // x rows a stage reads
-constexpr int RING = 6;               // x rows resident per channel
-constexpr int G_CH = SR * SW * 2 + 16;        // 272 bytes per g channel
-constexpr int X_ROW = 144;                    // 72 pixels
-constexpr int X_CH = RING * X_ROW + 16;       // 880 bytes per x channel
+constexpr int SR = 2;                         // output rows per stage
+constexpr int X_ROW = 144;                    // bytes of an x row in LDS: 66 pixels used
 constexpr int X_CPR = 8;                      // 8-pixel chunks per x row; 2 more pixels follow as one dword
+// By stride (1 or 2, the same along both axes). At stride 2 a stage of 2 x 32 output pixels reads 5 x 65 of x:
+// the rows are as long as at stride 1. They go to LDS with their even columns in front and the odd ones behind
+// (80 bytes on), so that the taps of a row are runs of consecutive pixels again: even[j], odd[j], even[j + 1].
+// (The stride-1 kernel on a gradient with zeros between its pixels did four times the work, and the copies
+// that made it: 64 -> 128 channels of 4 x 257 x 257 took 100 us.)
+template <int ST>
+struct Stage {
+  static constexpr int SW = 64 / ST;              // output columns per stage
+  static constexpr int XR = ST * (SR - 1) + 3;    // x rows a stage reads
+  static constexpr int NEW = ST * SR;             // of which this many are new; the others are the stage above's last
+  static constexpr int RING = XR + NEW;           // x rows resident per channel
+  static constexpr int G_CH = SR * SW * 2 + 16;   // bytes per g channel
+  static constexpr int X_CH = (RING * X_ROW) % 32 == 0 ? RING * X_ROW + 16 : RING * X_ROW + 32;  // per x channel: an odd multiple of 16
+};
+constexpr int X_ODD = 80;                         // stride 2: where the odd columns of a row start
 
 struct WgradParams {
   const uint16_t* x;  // (N, Cin, Din, Hin, Win)
@@ -122,16 +133,20 @@ __device__ __forceinline__ float sum_of_8(const u32x4& v) {
 // rows inside g (a convolution without padding over a tensor that holds its halo, tiles of whole
 // stages): the kernel is built without the element-wise border path, and its stage loop loads and
 // stores without conditions.
-template <int CGB, int CXB, int EVEN, bool FRAMED, bool F16 = false, bool ALLIN = false>
+template <int CGB, int CXB, int EVEN, bool FRAMED, bool F16 = false, bool ALLIN = false, int ST = 1>
 __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(WgradParams p) {
   constexpr int THREADS = wgrad_threads(CGB, CXB);
   constexpr int LEAD = EVEN == 2 ? 1 : 0;
   static_assert(!(FRAMED && EVEN != 1), "the framed input is read with even windows only");
+  static_assert(ST == 1 || (EVEN != 2 && !FRAMED && !ALLIN && CXB != 3), "stride 2 is built for plain 2-D tensors");
+  constexpr int SW = Stage<ST>::SW, XR = Stage<ST>::XR, NEW = Stage<ST>::NEW, RING = Stage<ST>::RING;
+  constexpr int G_CH = Stage<ST>::G_CH, X_CH = Stage<ST>::X_CH;
+  constexpr int G_CPR = SW / 8;  // chunks per g row
   constexpr int CWAVES = CGB * CXB * HALVES;  // wavefronts that own accumulators
   constexpr int GC = 32 * CGB, XC = 32 * CXB;
   constexpr int G_BYTES = GC * G_CH;          // one g buffer
-  constexpr int G_CHUNKS = GC * SR * (SW / 8);
-  constexpr int XP_CHUNKS = XC * 2 * X_CPR;   // one pair of x rows
+  constexpr int G_CHUNKS = GC * SR * G_CPR;
+  constexpr int XP_CHUNKS = XC * NEW * X_CPR;   // the new x rows of a stage
   constexpr int CHUNKS = G_CHUNKS + XP_CHUNKS;
   constexpr int ROUNDS = (CHUNKS + THREADS - 1) / THREADS;
   static_assert(G_CHUNKS % THREADS == 0, "a load round holds g chunks or x chunks, never both");
@@ -177,12 +192,12 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
   // is 8 pixels of a g row, the others 8 pixels of one of the two x rows of a pair.
   uint32_t c_goff[ROUNDS];  // byte offset from the origin of its tensor window
   uint32_t c_lds[ROUNDS];   // byte offset inside the g buffer / inside the x ring, row slot 0
-  uint32_t x_second = 0;    // bit rd: the chunk belongs to the second row of the pair
+  uint32_t x_row = 0;       // two bits per round: the chunk's row among the new ones
 #pragma unroll
   for (int rd = 0; rd < ROUNDS; ++rd) {
     const int q = tid + rd * THREADS;
     if (q < G_CHUNKS) {
-      const int c8 = q & 7, r = (q >> 3) % SR, ch = q / (8 * SR);
+      const int c8 = q % G_CPR, r = (q / G_CPR) % SR, ch = q / (G_CPR * SR);
       const int che = ch < cout_valid ? ch : cout_valid - 1;  // a channel past the last one reads the last
       c_goff[rd] = (uint32_t)((che * g_cs + (size_t)r * p.Wout + c8 * 8) * 2);
       c_lds[rd] = (uint32_t)(ch * G_CH + r * (SW * 2) + c8 * 16);
@@ -190,27 +205,28 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
       const int qx = q - G_CHUNKS;
       const int c8 = qx % X_CPR;
       const int rr = qx / X_CPR;
-      const int r2 = rr & 1, ch = rr >> 1;      // ch = kd * CIN_B + ci
+      const int r2 = rr % NEW, ch = rr / NEW;   // ch = kd * CIN_B + ci
       const int kd = ch / CIN_B, cib = ch - kd * CIN_B;
       const int ci = cib < cin_valid ? cib : cin_valid - 1;
       c_goff[rd] = (uint32_t)((ci * x_cs + kd * plane_x + (size_t)r2 * p.Win + c8 * 8) * 2);
-      c_lds[rd] = (uint32_t)(ch * X_CH + c8 * 16);
-      x_second |= (uint32_t)r2 << rd;
+      c_lds[rd] = (uint32_t)(ch * X_CH + c8 * (16 / ST));
+      x_row |= (uint32_t)r2 << (2 * rd);
     } else {
       c_goff[rd] = 0;
       c_lds[rd] = 0;
     }
   }
   // pixels 64, 65 of an x row (and 66, 67 of a window staged one pixel early): one or two dwords,
-  // carried by the first 2 * XC threads
-  const bool has_tail = tid < 2 * XC;
+  // carried by the first NEW * XC threads
+  static_assert(NEW * XC <= THREADS, "a thread carries one tail");
+  const bool has_tail = tid < NEW * XC;
   uint32_t t_goff = 0, t_lds = 0;
   if (has_tail) {
-    const int r2 = tid & 1, ch = tid >> 1;
+    const int r2 = tid % NEW, ch = tid / NEW;
     const int kd = ch / CIN_B, cib = ch - kd * CIN_B;
     const int ci = cib < cin_valid ? cib : cin_valid - 1;
-    t_goff = (uint32_t)((ci * x_cs + kd * plane_x + (size_t)r2 * p.Win + SW) * 2);
-    t_lds = (uint32_t)(ch * X_CH + SW * 2);
+    t_goff = (uint32_t)((ci * x_cs + kd * plane_x + (size_t)r2 * p.Win + 64) * 2);
+    t_lds = (uint32_t)(ch * X_CH + 128 / ST);
   }
   // the same x offsets inside the own tile (framed input)
   const size_t plane_t = (size_t)p.tn_h * p.tn_w, t_cs = plane_t * p.tn_d;
@@ -285,7 +301,8 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     u32x4 (&v)[ROUNDS] = sg.v;
     const int hp = cur.hp, ct = cur.ct, od = cur.od, n = cur.n;
     const int oh0 = hp * SR, ow0 = ct * SW;
-    const int id0 = od - p.pad_d, ih0 = oh0 - p.pad_h + 2 * xpair, iw0 = ow0 - p.pad_w - LEAD;
+    // first of the rows: of the new ones, or (xpair 0) as many rows further up, the last of which a first stage lacks
+    const int id0 = od - p.pad_d, ih0 = ST * oh0 - p.pad_h + XR - (xpair ? 1 : 2) * NEW, iw0 = ST * ow0 - p.pad_w - LEAD;
     const char* g_org = reinterpret_cast<const char*>(gb) +
                         2 * (((size_t)n * p.cout_total * p.Dout + od) * plane_g + (size_t)oh0 * p.Wout + ow0);
     const char* x_org = reinterpret_cast<const char*>(xb) +
@@ -293,7 +310,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
                              (ptrdiff_t)ih0 * p.Win + iw0);
     // (with LEAD the window's last dword holds one pixel more than is used; it shares its dword with one that is)
     const bool inside = ALLIN || (oh0 + SR <= p.Hout && ow0 + SW <= p.Wout && ih0 >= 0 &&
-                        ih0 + 2 <= p.Hin && iw0 >= 0 && iw0 + SW + 2 + LEAD <= p.Win && id0 >= 0 &&
+                        ih0 + NEW <= p.Hin && iw0 >= 0 && iw0 + 66 + LEAD <= p.Win && id0 >= 0 &&
                         id0 + KD <= p.Din);
     sg.masked = !inside;
     sg.odd = 0;
@@ -404,7 +421,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
         return ((1u << past) - 1u) & ~((1u << first) - 1u);
       };
       const int c8 = tid & 7;  // a round is a multiple of 8 chunks: the same in all of them
-      sg.g_cols = columns(ow0 + c8 * 8, 8, p.Wout);
+      sg.g_cols = columns(ow0 + (tid % G_CPR) * 8, 8, p.Wout);
       sg.x_cols = columns(iw0 + c8 * 8, 8, p.Win);
       sg.rows = 0;
       uint32_t over = 0;
@@ -415,10 +432,10 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
         const int q = tid + rd * THREADS;
         bool row_ok;
         if (g_round) {
-          row_ok = oh0 + ((q >> 3) % SR) < p.Hout;
+          row_ok = oh0 + (q / G_CPR) % SR < p.Hout;
         } else {
           const int rr = (q - G_CHUNKS) / X_CPR;
-          const int row = ih0 + (rr & 1), dd = id0 + (rr >> 1) / CIN_B;
+          const int row = ih0 + rr % NEW, dd = id0 + (rr / NEW) / CIN_B;
           row_ok = q < CHUNKS && row >= 0 && row < p.Hin && dd >= 0 && dd < p.Din;
         }
         const bool need = row_ok && (g_round ? sg.g_cols : sg.x_cols) != 0u;
@@ -456,12 +473,12 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
         }
       }
       if (has_tail) {
-        const int r2 = tid & 1, ch = tid >> 1;
+        const int r2 = tid % NEW, ch = tid / NEW;
         const int row = ih0 + r2, dd = id0 + ch / CIN_B;
         const uintptr_t at = reinterpret_cast<uintptr_t>(x_org) + t_goff;
         const uintptr_t down = at & ~(uintptr_t)3;
         const bool ok = dd >= 0 && dd < p.Din && row >= 0 && row < p.Hin;
-        sg.tail_cols = ok ? columns(iw0 + SW, 2 + 2 * LEAD, p.Win) : 0u;
+        sg.tail_cols = ok ? columns(iw0 + 64, 2 + 2 * LEAD, p.Win) : 0u;
         sg.tail = sg.tail_cols != 0u ? dword_at(down, p.x, p.x_end) : 0u;
         if (LEAD) sg.tail_b = (sg.tail_cols >> 2) != 0u ? dword_at(down + 4, p.x, p.x_end) : 0u;
         if (EVEN == 0) {
@@ -472,12 +489,12 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     }
   };
 
-  // Registers of a stage to LDS: g rows into g buffer `gbuf`, the x pair into ring rows
-  // `slot_a`, `slot_b`; the g chunks are added into the bias partials on the way.
+  // Registers of a stage to LDS: g rows into g buffer `gbuf`, the x rows into ring rows
+  // slot0, slot0 + 1, ..; the g chunks are added into the bias partials on the way.
   float bsum[ROUNDS];
 #pragma unroll
   for (int rd = 0; rd < ROUNDS; ++rd) bsum[rd] = 0.0f;
-  auto store_loads = [&](const Staged& sg, bool have_g, int gbuf, int slot_a, int slot_b, bool counted = true) {
+  auto store_loads = [&](const Staged& sg, bool have_g, int gbuf, int slot0, bool counted = true) {
     uint32_t g_keep[4], x_keep[4];
     if (!ALLIN && sg.masked) {
 #pragma unroll
@@ -510,12 +527,23 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
         *reinterpret_cast<u32x4*>(smem + gbuf * G_BYTES + c_lds[rd]) = val;
         if (bias_part != nullptr) bsum[rd] += counted ? sum_of_8<F16>(val) : 0.0f;
       } else if (q < CHUNKS) {
-        const int slot = ((x_second >> rd) & 1u) ? slot_b : slot_a;
-        *reinterpret_cast<u32x4*>(lds_x + c_lds[rd] + slot * X_ROW) = val;
+        int slot = slot0 + (int)((x_row >> (2 * rd)) & 3u);
+        if (slot >= RING) slot -= RING;
+        unsigned char* const at = lds_x + c_lds[rd] + slot * X_ROW;
+        if (ST == 1) {
+          *reinterpret_cast<u32x4*>(at) = val;
+        } else {
+          *reinterpret_cast<uint64_t*>(at) = (uint64_t)__builtin_amdgcn_perm(val.y, val.x, 0x05040100u) |
+                                             (uint64_t)__builtin_amdgcn_perm(val.w, val.z, 0x05040100u) << 32;
+          *reinterpret_cast<uint64_t*>(at + X_ODD) = (uint64_t)__builtin_amdgcn_perm(val.y, val.x, 0x07060302u) |
+                                                     (uint64_t)__builtin_amdgcn_perm(val.w, val.z, 0x07060302u) << 32;
+        }
       }
     }
     if (has_tail) {
-      unsigned char* at = lds_x + t_lds + ((tid & 1) ? slot_b : slot_a) * X_ROW;
+      int slot = slot0 + tid % NEW;
+      if (slot >= RING) slot -= RING;
+      unsigned char* at = lds_x + t_lds + slot * X_ROW;
       uint32_t t = sg.tail, tb = sg.tail_b;
       if (EVEN == 0) t = __builtin_amdgcn_alignbit(tb, t, (sg.odd >> 31) << 4);
       if (!ALLIN && sg.masked) {
@@ -539,15 +567,17 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
   // four x rows sit in ring rows base .. base + 3 (mod RING): first all its LDS reads
   // (read_group), then its matrix instructions (mfma_group), so that a stage can ask for both
   // of its groups before the first matrix instruction and meets the LDS latency once.
+  constexpr int GROUPS = SW / 16 / HALVES;
   struct Frags {
     u32x4 a[SR];
     u32x4 d[XR];
     uint32_t d4[XR], d5[XR];
+    u32x4 odd[XR];  // stride 2
   };
   auto read_group = [&](Frags& f, int gbuf, int base, int cgi) __attribute__((always_inline)) {
     const unsigned char* gb = smem + gbuf * G_BYTES + (cb * 32 + ln) * G_CH + kgp * 16;
     const unsigned char* xb = lds_x + (ib * 32 + ln) * X_CH + kgp * 16;
-    const int cg = half * (SW / 16 / HALVES) + cgi;  // 16-pixel column group of this wavefront
+    const int cg = half * GROUPS + cgi;  // 16-pixel column group of this wavefront
 #pragma unroll
     for (int r = 0; r < SR; ++r) f.a[r] = *reinterpret_cast<const u32x4*>(gb + r * (SW * 2) + cg * 32);
 #pragma unroll
@@ -558,6 +588,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
       f.d4[rho] = *reinterpret_cast<const uint32_t*>(xb + slot * X_ROW + cg * 32 + 16);
       f.d5[rho] = 0u;
       if (LEAD) f.d5[rho] = *reinterpret_cast<const uint32_t*>(xb + slot * X_ROW + cg * 32 + 20);
+      if (ST == 2) f.odd[rho] = *reinterpret_cast<const u32x4*>(xb + slot * X_ROW + X_ODD + cg * 32);
     }
   };
   auto mfma_group = [&](Frags& f) __attribute__((always_inline)) {
@@ -584,11 +615,11 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
       s3.z = __builtin_amdgcn_alignbit(d4, d.w, 16);
       s3.w = __builtin_amdgcn_alignbit(d5, d4, 16);
       const bf16x8 b0 = __builtin_bit_cast(bf16x8, LEAD ? s1 : d);
-      const bf16x8 b1 = __builtin_bit_cast(bf16x8, LEAD ? s2 : s1);
-      const bf16x8 b2 = __builtin_bit_cast(bf16x8, LEAD ? s3 : s2);
+      const bf16x8 b1 = __builtin_bit_cast(bf16x8, ST == 2 ? f.odd[rho] : LEAD ? s2 : s1);
+      const bf16x8 b2 = __builtin_bit_cast(bf16x8, ST == 2 ? s1 : LEAD ? s3 : s2);
 #pragma unroll
       for (int r = 0; r < SR; ++r) {
-        const int kh = rho - r;
+        const int kh = rho - ST * r;
         if (kh >= 0 && kh < 3) {
           if (F16) {
             const f16x8 ah = __builtin_bit_cast(f16x8, a[r]);
@@ -610,20 +641,22 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     mfma_group(f);
   };
 
-  // Stage k of this workgroup reads ring rows base_k .. base_k + 3 with base_k = 2k mod 6:
-  // its first two rows are where the stage before put its new rows (base_k-1 + 2, + 3), its
-  // new rows go to base_k + 2, + 3. A stage that does not continue the strip of the stage
-  // before fetches its first two rows itself, into those same ring rows.
-  static_assert(SW / 16 / HALVES == 2, "the stage loop is written for two column groups per wavefront");
+  // Stage k of this workgroup reads ring rows base_k .. base_k + XR - 1 with base_k = NEW k mod RING: its
+  // first OLD rows are the last ones the stage before read, its new rows go behind them. A stage that does
+  // not continue the strip of the stage before fetches the old rows itself, into those same ring rows (as
+  // many rows as the new ones at stride 2, of which the last is the old one: the others go to ring rows
+  // that nobody reads).
+  static_assert(GROUPS == 2 || (GROUPS == 1 && !ALLIN), "the stage loop is written for one or two column groups per wavefront");
   auto wrap = [](int v) { return v >= RING ? v - RING : v; };
   if (s_begin < s_end) {
     Staged stg;
     int gbuf = 0, base = 0;
     Cursor c_next = decode(s_begin);  // stage whose loads are issued next
     issue_loads(stg, c_next, true, 1);
-    store_loads(stg, true, 0, 2, 3);
+    constexpr int OLD = XR - NEW;  // rows a stage shares with the one above
+    store_loads(stg, true, 0, OLD);
     issue_loads(stg, c_next, false, 0);
-    store_loads(stg, false, 0, 0, 1);
+    store_loads(stg, false, 0, (OLD - NEW + RING) % RING);
     if constexpr (ALLIN) {
       // The loads of a stage are issued, and the registers of the stage before stored, in EVERY
       // stage: the cursor stops at the workgroup's last stage, which the last two stages fetch
@@ -649,7 +682,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
       for (long long st = s_begin; st < s_end; ++st) {
         Frags f0, f1;
         if (stage_first) {
-          store_loads(stg, true, gbuf ^ 1, wrap(base + 4), wrap(base + 5), st + 1 < s_end);
+          store_loads(stg, true, gbuf ^ 1, wrap(base + XR), st + 1 < s_end);
           issue_loads(stg, c_next, true, 1);
         }
         if (wave < CWAVES) {
@@ -659,7 +692,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
           if (CWAVES == 8) mfma_group(f1);
         }
         if (!stage_first) {
-          store_loads(stg, true, gbuf ^ 1, wrap(base + 4), wrap(base + 5), st + 1 < s_end);
+          store_loads(stg, true, gbuf ^ 1, wrap(base + XR), st + 1 < s_end);
           issue_loads(stg, c_next, true, 1);
         }
         if (CWAVES != 8 && wave < CWAVES) mfma_group(f1);
@@ -669,7 +702,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
           // the next stage starts a new strip: its first two x rows, on the spot
           Staged top;
           issue_loads(top, c_store, false, 0);
-          store_loads(top, false, 0, wrap(base + 2), wrap(base + 3));
+          store_loads(top, false, 0, wrap(base + OLD));
           // These loads have all been stored, but the tail's under a per-lane condition: where
           // the compiler cannot see a load waited for on every path, it waits at the loop's end,
           // and that wait takes the stage's own loads with it. vmcnt(0), said once, here:
@@ -677,7 +710,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
           __syncthreads();
         }
         advance(c_store);
-        base = wrap(base + 2);
+        base = wrap(base + NEW);
         gbuf ^= 1;
       }
     } else {
@@ -690,28 +723,28 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
       __syncthreads();
       for (long long st = s_begin; st < s_end; ++st) {
         if (wave < CWAVES) compute_group(gbuf, base, 0);
-        if (st + 1 < s_end) store_loads(stg, true, gbuf ^ 1, wrap(base + 4), wrap(base + 5));
+        if (st + 1 < s_end) store_loads(stg, true, gbuf ^ 1, wrap(base + XR));
         if (st + 2 < s_end) {
           issue_loads(stg, c_next, true, 1);
           advance(c_next);
         }
-        if (wave < CWAVES) compute_group(gbuf, base, 1);
+        if (GROUPS == 2 && wave < CWAVES) compute_group(gbuf, base, 1);
         __syncthreads();
         if (st + 1 < s_end && c_store.hp == 0) {
           // the next stage starts a new strip: its first two x rows, on the spot
           Staged top;
           issue_loads(top, c_store, false, 0);
-          store_loads(top, false, 0, wrap(base + 2), wrap(base + 3));
+          store_loads(top, false, 0, wrap(base + OLD));
           __syncthreads();
         }
         advance(c_store);
-        base = wrap(base + 2);
+        base = wrap(base + NEW);
         gbuf ^= 1;
       }
     }
   }
 
-  // bias partial of this workgroup: the 16 lanes that carried a channel's chunks add up
+  // bias partial of this workgroup: the lanes that carried a channel's chunks add up
   const size_t slot = (size_t)block * gridDim.x + blockIdx.x;
   if (bias_part != nullptr) {
 #pragma unroll
@@ -719,11 +752,9 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
       const int q = tid + rd * THREADS;
       if (rd * THREADS < G_CHUNKS) {  // rounds that hold g chunks (whole rounds: THREADS divides G_CHUNKS)
         float s = bsum[rd];
-        s += __shfl_xor(s, 8, 64);
-        s += __shfl_xor(s, 4, 64);
-        s += __shfl_xor(s, 2, 64);
-        s += __shfl_xor(s, 1, 64);
-        if (q < G_CHUNKS && (tid & 15) == 0) bias_part[slot * GC + q / (8 * SR)] = s;
+#pragma unroll
+        for (int off = SR * G_CPR / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        if (q < G_CHUNKS && tid % (SR * G_CPR) == 0) bias_part[slot * GC + q / (SR * G_CPR)] = s;
       }
     }
   }
@@ -878,8 +909,10 @@ int cu_count() {
   return n;
 }
 
+int stage_columns(const ConvGeom& g) { return g.s[2] == 2 ? Stage<2>::SW : Stage<1>::SW; }
 long long stage_count(const ConvGeom& g) {
-  return g.batch * g.out[0] * ((g.out[1] + SR - 1) / SR) * ((g.out[2] + SW - 1) / SW);
+  const int sw = stage_columns(g);
+  return g.batch * g.out[0] * ((g.out[1] + SR - 1) / SR) * ((g.out[2] + sw - 1) / sw);
 }
 
 // Channel blocking. A workgroup accumulates a block of GC output x CIN_B input channels (32 or 64 each; with a
@@ -901,8 +934,9 @@ bool covered(const ConvGeom& g) {
   if (g.groups != 1) return false;
   if (g.k[1] != 3 || g.k[2] != 3 || (g.k[0] != 1 && g.k[0] != 3)) return false;
   if (g.k[0] == 1 && g.in[0] != 1) return false;
+  const bool strided = g.s[1] == 2 && g.s[2] == 2 && g.k[0] == 1;
   for (int a = 0; a < 3; ++a)
-    if (g.s[a] != 1 || g.d[a] != 1) return false;
+    if ((g.s[a] != 1 && !(strided && a > 0)) || g.d[a] != 1) return false;
   if (g.cin <= 0 || g.cout <= 0) return false;
   // per-lane byte offsets inside one batch entry are 32-bit
   const size_t xs = (size_t)g.cin * g.in[0] * g.in[1] * g.in[2] * 2;
@@ -941,11 +975,17 @@ Plan plan_of(const ConvGeom& g, int parts) {
 }
 
 template <int CGB, int CXB>
-int launch(const WgradParams& p, int even, bool f16, bool all_inside, dim3 grid, hipStream_t s, const char* who) {
+int launch(const WgradParams& p, int even, bool f16, bool all_inside, int stride, dim3 grid, hipStream_t s, const char* who) {
   constexpr int THREADS = wgrad_threads(CGB, CXB);
-  const size_t lds = 2 * (size_t)(32 * CGB * G_CH) + (size_t)(32 * CXB * X_CH);
-  void (*kern)(WgradParams);
-  if (f16)  // never framed (checked by the caller)
+  const size_t lds = stride == 2 ? 2 * (size_t)(32 * CGB * Stage<2>::G_CH) + (size_t)(32 * CXB * Stage<2>::X_CH)
+                                 : 2 * (size_t)(32 * CGB * Stage<1>::G_CH) + (size_t)(32 * CXB * Stage<1>::X_CH);
+  void (*kern)(WgradParams) = nullptr;
+  if (stride == 2) {
+    if constexpr (CXB != 3) {
+      if (f16) kern = even == 1 ? &wgrad3x3_mfma_kernel<CGB, CXB, 1, false, true, false, 2> : &wgrad3x3_mfma_kernel<CGB, CXB, 0, false, true, false, 2>;
+      else kern = even == 1 ? &wgrad3x3_mfma_kernel<CGB, CXB, 1, false, false, false, 2> : &wgrad3x3_mfma_kernel<CGB, CXB, 0, false, false, false, 2>;
+    }
+  } else if (f16)  // never framed (checked by the caller)
     kern = even == 1 ? &wgrad3x3_mfma_kernel<CGB, CXB, 1, false, true>
                      : (even == 2 ? &wgrad3x3_mfma_kernel<CGB, CXB, 2, false, true> : &wgrad3x3_mfma_kernel<CGB, CXB, 0, false, true>);
   else if (p.xt != nullptr)
@@ -994,7 +1034,8 @@ size_t mfma_wgrad_workspace(const ConvGeom& g, int dtype) {
 // inside the bands that the frame holds.
 bool mfma_wgrad_frame_ok(const ConvGeom& g, const int tlo[3], const int tn[3]) {
   if (g.in[2] % 2 != 0 || g.p[2] % 2 != 0 || g.out[2] % 2 != 0 || tn[2] % 2 != 0) return false;
-  if (!covered(g)) return false;
+  if (!covered(g) || g.s[2] != 1) return false;
+  constexpr int SW = Stage<1>::SW;
   const Plan plan = plan_of(g, 1);  // the framed input is read by a single block of exactly its width
   if (g.cin * plan.KD != (int)plan.XC() || g.cout != (int)plan.GC()) return false;
   int blo[3], bhi[3];
@@ -1069,10 +1110,11 @@ int mfma_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom
   p.Dout = g.out[0]; p.Hout = g.out[1]; p.Wout = g.out[2];
   p.pad_d = g.p[0]; p.pad_h = g.p[1]; p.pad_w = g.p[2];
   p.row_pairs = (g.out[1] + SR - 1) / SR;
-  p.col_tiles = (g.out[2] + SW - 1) / SW;
+  p.col_tiles = (g.out[2] + stage_columns(g) - 1) / stage_columns(g);
   p.total_stages = stage_count(g);
   // Every stage whole and every window inside x: the kernel without the border path (see ALLIN).
-  const bool all_inside = even == 1 && xt == nullptr && g.p[0] == 0 && g.p[1] == 0 && g.p[2] == 0 &&
+  constexpr int SW = Stage<1>::SW;
+  const bool all_inside = g.s[2] == 1 && even == 1 && xt == nullptr && g.p[0] == 0 && g.p[1] == 0 && g.p[2] == 0 &&
                           g.out[1] % SR == 0 && g.out[2] % SW == 0 && g.out[1] + 2 <= g.in[1] &&
                           g.out[2] + 2 <= g.in[2] && g.out[0] - 1 + g.k[0] <= g.in[0];
   p.xt = static_cast<const uint16_t*>(xt);
@@ -1081,11 +1123,11 @@ int mfma_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom
   JG_REQUIRE(plan.blocks() < 65536, "%s: too many channels", who);
   const dim3 grid((unsigned)plan.wgs, (unsigned)plan.blocks());
   int rc;
-  if (plan.cgb == 2 && plan.cxb == 2) rc = launch<2, 2>(p, even, f16, all_inside, grid, s, who);
-  else if (plan.cgb == 1 && plan.cxb == 3) rc = launch<1, 3>(p, even, f16, all_inside, grid, s, who);
-  else if (plan.cgb == 1 && plan.cxb == 1) rc = launch<1, 1>(p, even, f16, all_inside, grid, s, who);
-  else if (plan.cgb == 2 && plan.cxb == 1) rc = launch<2, 1>(p, even, f16, all_inside, grid, s, who);
-  else rc = launch<1, 2>(p, even, f16, all_inside, grid, s, who);
+  if (plan.cgb == 2 && plan.cxb == 2) rc = launch<2, 2>(p, even, f16, all_inside, g.s[2], grid, s, who);
+  else if (plan.cgb == 1 && plan.cxb == 3) rc = launch<1, 3>(p, even, f16, all_inside, g.s[2], grid, s, who);
+  else if (plan.cgb == 1 && plan.cxb == 1) rc = launch<1, 1>(p, even, f16, all_inside, g.s[2], grid, s, who);
+  else if (plan.cgb == 2 && plan.cxb == 1) rc = launch<2, 1>(p, even, f16, all_inside, g.s[2], grid, s, who);
+  else rc = launch<1, 2>(p, even, f16, all_inside, g.s[2], grid, s, who);
   if (rc) return rc;
   JG_CHECK_LAUNCH(who);
 
