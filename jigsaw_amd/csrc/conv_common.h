@@ -58,4 +58,15 @@ int mfma_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom
 // three for fp32, two for fp16. The operand layout of the split mode of the MFMA kernels.
 int split_parts_bf16(uint16_t* dst, const void* src, int src_dtype, size_t batch, size_t per_batch, hipStream_t s);
 
+// Loads from an address worked out as a number (rounded down to a dword, chosen per lane): as plain pointers
+// these would be flat accesses, which count as LDS traffic too and make the compiler wait for each of them.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define JG_GLOBAL __attribute__((address_space(1)))
+#else
+#define JG_GLOBAL
+#endif
+typedef uint32_t jg_u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ jg_u32x4_a4 load_16_bytes_at(uintptr_t at) { return *(const JG_GLOBAL jg_u32x4_a4*)at; }
+__device__ __forceinline__ uint32_t load_4_bytes_at(uintptr_t at) { return *(const JG_GLOBAL uint32_t*)at; }
+
 }  // namespace jg

@@ -399,7 +399,8 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   const uint32_t t_off_t = (uint32_t)(((size_t)g8 * 8 * chan_stride_t + (size_t)t_row * p.tn_w + t_col) * 2);
   uint32_t stg[8][4];
   bool stg_masked = false;    // wave-uniform: the staged window sticks out of the tensor
-  uint32_t stg_mask = 0xffu;  // this task's pixels inside the tensor (one bit each), where stg_masked
+  const char* stg_origin = nullptr;  // its origin (wave-uniform)
+  uint32_t stg_mask = 0xffu;  // this task's pixels inside the tensor (one bit each), where stg_masked; bit 8: not loaded yet
   uint32_t stg_odd = 0;       // not EVEN: one bit per channel, the task starts on the upper half of a dword
 
   struct TileCoord {
@@ -539,70 +540,69 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
       }
     }
     stg_masked = !interior;
+    stg_origin = origin;
     if (!has_task) return;
-    const char* a = origin + t_off;
-    if (interior) {
-      if (EVEN) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const u32x4_a4 v = *reinterpret_cast<const u32x4_a4*>(a + (size_t)c * chan_b);
-          stg[c][0] = v.x; stg[c][1] = v.y; stg[c][2] = v.z; stg[c][3] = v.w;
-        }
-      } else {
-        const char* down = reinterpret_cast<const char*>(reinterpret_cast<uintptr_t>(origin) & ~(uintptr_t)3);  // uniform
-        uint32_t off = t_off + (uint32_t)(reinterpret_cast<uintptr_t>(origin) & 3);
-        stg_odd = 0;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const u32x4_a4 v = *reinterpret_cast<const u32x4_a4*>(down + (off & ~3u));
-          stg[c][0] = v.x; stg[c][1] = v.y; stg[c][2] = v.z; stg[c][3] = v.w;
-          stg_odd |= ((off >> 1) & 1u) << c;
-          off += chan_b;
-        }
-      }
-    } else {
+    // One set of loads for every window, from addresses that differ: a load under a condition leaves its register
+    // with two possible values where the paths meet, and the compiler then waits for it right there, half a stage
+    // before it is wanted (a border window took the whole latency of memory that way).
+    uintptr_t from = reinterpret_cast<uintptr_t>(origin);  // wave-uniform where the window lies inside the tensor
+    uint32_t off = t_off;
+    uint32_t step = chan_b;
+    int steps = 8;
+    if (!interior) {
       // A window that sticks out of the tensor, or whose 16 channels do (a ragged last step). A task reads
       // its 16 bytes wherever they lie inside the tensor, also past the end of its row; store_stage clears
       // the pixels that are not the row's. Tasks without any pixel of the tensor read the prepared weights
-      // instead, so that no load stands under a condition. What is left are the tasks whose bytes reach
-      // over the tensor's own ends: those go dword by dword.
+      // instead, and so do those whose bytes reach over the tensor's own ends: store_stage fetches these.
       const int ih = ih0 + t_row, iw = iw0 + t_col;
       const bool row_ok = depth_ok && ih >= 0 && ih < p.Hin && cvalid > 0;
       const int first = max(0, min(8, -iw)), past = max(0, min(8, p.Win - iw));
       stg_mask = row_ok ? ((1u << past) - 1u) & ~((1u << first) - 1u) : 0u;
       // (not EVEN: the task before takes its last pixel from this one's first dword)
       const bool need = EVEN ? stg_mask != 0u : row_ok && iw - 1 < p.Win && iw + 8 > 0;
+      const char* a = origin + t_off;
       const uint32_t span = (uint32_t)(min(cvalid, 8) - 1) * chan_b;
       const bool fits = a >= reinterpret_cast<const char*>(p.x) && a + (size_t)span + 16 <= p.x_end;
-      const char* from = need && fits ? a : reinterpret_cast<const char*>(p.wprep);
-      const uint32_t step = need && fits ? chan_b : 0u;
-      uint32_t off = 0;
+      if (need && !fits) stg_mask |= 0x100u;
+      from = reinterpret_cast<uintptr_t>(need && fits ? a : reinterpret_cast<const char*>(p.wprep));
+      step = need && fits ? chan_b : 0u;
+      steps = cvalid;
+      off = 0;
+    }
+    if (!EVEN) {
+      off += (uint32_t)(from & 3);
+      from &= ~(uintptr_t)3;
       stg_odd = 0;
+    }
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const uintptr_t at = reinterpret_cast<uintptr_t>(from) + off;
-        const u32x4_a4 v = *reinterpret_cast<const u32x4_a4*>(EVEN ? at : at & ~(uintptr_t)3);
-        stg[c][0] = v.x; stg[c][1] = v.y; stg[c][2] = v.z; stg[c][3] = v.w;
-        if (!EVEN) stg_odd |= (uint32_t)((at >> 1) & 1) << c;
-        off += c + 1 < cvalid ? step : 0u;
-      }
-      if (__builtin_amdgcn_ballot_w64(need && !fits) != 0 && need && !fits) {
-        stg_odd = 0;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const uintptr_t at = reinterpret_cast<uintptr_t>(a) + (uint32_t)min(c, cvalid - 1) * (size_t)chan_b;
-          const char* d = reinterpret_cast<const char*>(at & ~(uintptr_t)3);
-          stg_odd |= (uint32_t)((at >> 1) & 1) << c;
-#pragma unroll
-          for (int j = 0; j < 4; ++j)  // a dword that holds a pixel of the tensor
-            stg[c][j] = d + 4 * j + 3 >= reinterpret_cast<const char*>(p.x) && d + 4 * j < p.x_end ? *reinterpret_cast<const uint32_t*>(d + 4 * j) : 0u;
-        }
-      }
+    for (int c = 0; c < 8; ++c) {
+      const u32x4_a4 v = jg::load_16_bytes_at(from + (EVEN ? off : off & ~3u));
+      stg[c][0] = v.x; stg[c][1] = v.y; stg[c][2] = v.z; stg[c][3] = v.w;
+      if (!EVEN) stg_odd |= ((off >> 1) & 1u) << c;
+      off += c + 1 < steps ? step : 0u;
     }
   };
 
   auto store_stage = [&](int buf, int stage) {  // stage: counted over this workgroup's tiles
     if (!has_task) return;
+    if (stg_masked && __builtin_amdgcn_ballot_w64((stg_mask & 0x100u) != 0) != 0) {
+      // a task whose bytes reach over the tensor's ends (the first and last rows of the first and last channel):
+      // dword by dword, those that hold a pixel of the tensor
+      if ((stg_mask & 0x100u) != 0) {
+        const int cvalid = p.C - ((stage % p.nc16) * CK) % p.Cp - g8 * 8;
+        const char* a = stg_origin + t_off;
+        stg_odd = 0;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const uintptr_t at = reinterpret_cast<uintptr_t>(a) + (uint32_t)min(c, cvalid - 1) * (size_t)chan_b;
+          const uintptr_t d = at & ~(uintptr_t)3;
+          stg_odd |= (uint32_t)((at >> 1) & 1) << c;
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            stg[c][j] = d + 4 * j + 3 >= reinterpret_cast<uintptr_t>(p.x) && d + 4 * j < reinterpret_cast<uintptr_t>(p.x_end) ? jg::load_4_bytes_at(d + 4 * j) : 0u;
+        }
+      }
+    }
     if (p.Cp != p.C) {  // uniform: zero the channels of this step that do not exist
       const int cvalid = p.C - ((stage % p.nc16) * CK) % p.Cp - g8 * 8;
 #pragma unroll

@@ -265,6 +265,8 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     // chunks all have the same columns), rounds whose row exists (one bit each), pixels of the tail
     bool masked;
     uint32_t g_cols, x_cols, rows, tail_cols;
+    uint32_t over;  // rounds (bit 31: the tail) whose bytes reach over the tensor's ends and are not loaded yet
+    const char *g_org, *x_org;
   };
 
   // Loads of one stage into `v`: its two g rows (want_g) and one pair of its x rows
@@ -385,50 +387,34 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
         return;
       }
     }
-    if (inside) {
-      // Every lane loads in every round it is asked for (the lanes past the last chunk and
-      // those without a tail read offset 0 of the window, which is there): a load under a
-      // per-lane condition merges the register with its old value, and the wait the
-      // compiler puts before such a merge stands behind this stage's loads, which are
-      // still in flight then.
+    // One set of loads for every stage, from addresses that differ: a load under a condition leaves its register with
+    // two possible values where the paths meet, and the compiler then waits for it right there instead of where it
+    // is stored, half a stage later. Every lane loads in every round it is asked for (the lanes past the last chunk
+    // and those without a tail read offset 0 of the window, or the workspace).
+    uintptr_t at[ROUNDS];
+    uintptr_t t_at = reinterpret_cast<uintptr_t>(x_org) + t_goff;
 #pragma unroll
-      for (int rd = 0; rd < ROUNDS; ++rd) {
-        const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;  // THREADS divides G_CHUNKS
-        if (!want_g && g_round) continue;
-        const uintptr_t at = reinterpret_cast<uintptr_t>(g_round ? g_org : x_org) + c_goff[rd];
-        if (EVEN == 0) {
-          v[rd] = *reinterpret_cast<const u32x4_a4*>(at & ~(uintptr_t)3);
-          sg.next[rd] = *reinterpret_cast<const uint32_t*>((at + 14) & ~(uintptr_t)3);
-          sg.odd |= (uint32_t)((at >> 1) & 1) << rd;
-        } else {
-          v[rd] = *reinterpret_cast<const u32x4_a4*>(at);
-        }
-      }
-      const uintptr_t at = reinterpret_cast<uintptr_t>(x_org) + t_goff;
-      sg.tail = *reinterpret_cast<const uint32_t*>(at & ~(uintptr_t)3);
-      if (LEAD) sg.tail_b = *reinterpret_cast<const uint32_t*>(at + 4);
-      if (EVEN == 0) {
-        sg.tail_b = *reinterpret_cast<const uint32_t*>((at + 2) & ~(uintptr_t)3);
-        sg.odd |= (uint32_t)((at >> 1) & 1) << 31;
-      }
-    } else {
+    for (int rd = 0; rd < ROUNDS; ++rd) at[rd] = reinterpret_cast<uintptr_t>((rd + 1) * THREADS <= G_CHUNKS ? g_org : x_org) + c_goff[rd];
+    if (!inside) {
       // A stage at an edge. A chunk is read wherever its bytes lie inside its tensor, also past the end of its
       // row; store_loads clears the pixels that are not the row's. A chunk without any pixel of the tensor reads
-      // the workspace instead, so that no load stands under a condition; what is left are the few chunks whose
-      // bytes reach over the tensor's own ends, which go dword by dword.
+      // the workspace instead, and so do the few whose bytes reach over the tensor's own ends: store_loads
+      // fetches these.
       auto columns = [](int col, int count, int cols) {  // of the pixels col .. col + count - 1, those in [0, cols)
         const int first = max(0, min(count, -col)), past = max(0, min(count, cols - col));
         return ((1u << past) - 1u) & ~((1u << first) - 1u);
       };
+      const uintptr_t safe = reinterpret_cast<uintptr_t>(p.part);
       const int c8 = tid & 7;  // a round is a multiple of 8 chunks: the same in all of them
       sg.g_cols = columns(ow0 + (tid % G_CPR) * 8, 8, p.Wout);
       sg.x_cols = columns(iw0 + c8 * 8, 8, p.Win);
       sg.rows = 0;
-      uint32_t over = 0;
+      sg.over = 0;
+      sg.g_org = g_org;
+      sg.x_org = x_org;
 #pragma unroll
       for (int rd = 0; rd < ROUNDS; ++rd) {
         const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;
-        if (!want_g && g_round) continue;
         const int q = tid + rd * THREADS;
         bool row_ok;
         if (g_round) {
@@ -439,52 +425,64 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
           row_ok = q < CHUNKS && row >= 0 && row < p.Hin && dd >= 0 && dd < p.Din;
         }
         const bool need = row_ok && (g_round ? sg.g_cols : sg.x_cols) != 0u;
+        const bool fits = at[rd] >= reinterpret_cast<uintptr_t>(g_round ? p.g : p.x) &&
+                          at[rd] + 16 <= reinterpret_cast<uintptr_t>(g_round ? p.g_end : p.x_end);
         sg.rows |= (need ? 1u : 0u) << rd;
-        const char* a = (g_round ? g_org : x_org) + c_goff[rd];
-        const bool fits = a >= reinterpret_cast<const char*>(g_round ? p.g : p.x) && a + 16 <= (g_round ? p.g_end : p.x_end);
-        over |= (need && !fits ? 1u : 0u) << rd;
-        const uintptr_t at = reinterpret_cast<uintptr_t>(need && fits ? a : reinterpret_cast<const char*>(p.part));
-        v[rd] = *reinterpret_cast<const u32x4_a4*>(at & ~(uintptr_t)3);
-        if (EVEN == 0) {
-          sg.next[rd] = *reinterpret_cast<const uint32_t*>((at + 14) & ~(uintptr_t)3);
-          sg.odd |= (uint32_t)((at >> 1) & 1) << rd;
-        }
+        sg.over |= (need && !fits ? 1u : 0u) << rd;
+        at[rd] = need && fits ? at[rd] : safe;
       }
-      auto dword_at = [](uintptr_t at, const void* begin, const char* end) {  // 0 where it holds no pixel of the tensor
-        return at + 4 > reinterpret_cast<uintptr_t>(begin) && at < reinterpret_cast<uintptr_t>(end) ? *reinterpret_cast<const uint32_t*>(at) : 0u;
-      };
-      if (__builtin_amdgcn_ballot_w64(over != 0u) != 0) {
+      const int row = ih0 + tid % NEW, dd = id0 + (tid / NEW) / CIN_B;
+      const bool ok = has_tail && dd >= 0 && dd < p.Din && row >= 0 && row < p.Hin;
+      sg.tail_cols = ok ? columns(iw0 + 64, 2 + 2 * LEAD, p.Win) : 0u;
+      const bool fits = t_at >= reinterpret_cast<uintptr_t>(p.x) && t_at + 4 + 4 * LEAD <= reinterpret_cast<uintptr_t>(p.x_end);
+      sg.over |= (sg.tail_cols != 0u && !fits ? 1u : 0u) << 31;
+      t_at = sg.tail_cols != 0u && fits ? t_at : safe;
+    }
 #pragma unroll
-        for (int rd = 0; rd < ROUNDS; ++rd) {
-          if (((over >> rd) & 1u) == 0) continue;
-          const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;
-          const void* begin = g_round ? p.g : p.x;
-          const char* end = g_round ? p.g_end : p.x_end;
-          const uintptr_t at = reinterpret_cast<uintptr_t>((g_round ? g_org : x_org) + c_goff[rd]);
-          const uintptr_t down = at & ~(uintptr_t)3;
-          v[rd].x = dword_at(down, begin, end);
-          v[rd].y = dword_at(down + 4, begin, end);
-          v[rd].z = dword_at(down + 8, begin, end);
-          v[rd].w = dword_at(down + 12, begin, end);
-          if (EVEN == 0) {
-            sg.next[rd] = dword_at((at + 14) & ~(uintptr_t)3, begin, end);
-            sg.odd = (sg.odd & ~(1u << rd)) | ((uint32_t)((at >> 1) & 1) << rd);
-          }
-        }
+    for (int rd = 0; rd < ROUNDS; ++rd) {
+      const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;  // THREADS divides G_CHUNKS
+      if (!want_g && g_round) continue;
+      v[rd] = jg::load_16_bytes_at(EVEN == 0 ? at[rd] & ~(uintptr_t)3 : at[rd]);
+      if (EVEN == 0) {
+        sg.next[rd] = jg::load_4_bytes_at((at[rd] + 14) & ~(uintptr_t)3);
+        sg.odd |= (uint32_t)((at[rd] >> 1) & 1) << rd;
       }
-      if (has_tail) {
-        const int r2 = tid % NEW, ch = tid / NEW;
-        const int row = ih0 + r2, dd = id0 + ch / CIN_B;
-        const uintptr_t at = reinterpret_cast<uintptr_t>(x_org) + t_goff;
-        const uintptr_t down = at & ~(uintptr_t)3;
-        const bool ok = dd >= 0 && dd < p.Din && row >= 0 && row < p.Hin;
-        sg.tail_cols = ok ? columns(iw0 + 64, 2 + 2 * LEAD, p.Win) : 0u;
-        sg.tail = sg.tail_cols != 0u ? dword_at(down, p.x, p.x_end) : 0u;
-        if (LEAD) sg.tail_b = (sg.tail_cols >> 2) != 0u ? dword_at(down + 4, p.x, p.x_end) : 0u;
-        if (EVEN == 0) {
-          sg.tail_b = sg.tail_cols != 0u ? dword_at((at + 2) & ~(uintptr_t)3, p.x, p.x_end) : 0u;
-          sg.odd |= (uint32_t)((at >> 1) & 1) << 31;
-        }
+    }
+    sg.tail = jg::load_4_bytes_at(t_at & ~(uintptr_t)3);
+    if (LEAD) sg.tail_b = jg::load_4_bytes_at(t_at + 4);
+    if (EVEN == 0) {
+      sg.tail_b = jg::load_4_bytes_at((t_at + 2) & ~(uintptr_t)3);
+      sg.odd |= (uint32_t)((t_at >> 1) & 1) << 31;
+    }
+  };
+  // The chunks of an edge stage whose bytes reach over the ends of their tensor: dword by dword, those that hold
+  // a pixel of it.
+  auto fetch_over = [&](Staged& sg, bool have_g) {
+    auto dword_at = [](uintptr_t at, const void* begin, const char* end) {
+      return at + 4 > reinterpret_cast<uintptr_t>(begin) && at < reinterpret_cast<uintptr_t>(end) ? jg::load_4_bytes_at(at) : 0u;
+    };
+#pragma unroll
+    for (int rd = 0; rd < ROUNDS; ++rd) {
+      const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;
+      if ((!have_g && g_round) || ((sg.over >> rd) & 1u) == 0) continue;
+      const void* begin = g_round ? p.g : p.x;
+      const char* end = g_round ? p.g_end : p.x_end;
+      const uintptr_t at = reinterpret_cast<uintptr_t>(g_round ? sg.g_org : sg.x_org) + c_goff[rd];
+      const uintptr_t down = at & ~(uintptr_t)3;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sg.v[rd][j] = dword_at(down + 4 * j, begin, end);
+      if (EVEN == 0) {
+        sg.next[rd] = dword_at((at + 14) & ~(uintptr_t)3, begin, end);
+        sg.odd = (sg.odd & ~(1u << rd)) | ((uint32_t)((at >> 1) & 1) << rd);
+      }
+    }
+    if ((sg.over >> 31) != 0) {
+      const uintptr_t at = reinterpret_cast<uintptr_t>(sg.x_org) + t_goff;
+      sg.tail = dword_at(at & ~(uintptr_t)3, p.x, p.x_end);
+      if (LEAD) sg.tail_b = dword_at(at + 4, p.x, p.x_end);
+      if (EVEN == 0) {
+        sg.tail_b = dword_at((at + 2) & ~(uintptr_t)3, p.x, p.x_end);
+        sg.odd = (sg.odd & 0x7fffffffu) | ((uint32_t)((at >> 1) & 1) << 31);
       }
     }
   };
@@ -494,9 +492,10 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
   float bsum[ROUNDS];
 #pragma unroll
   for (int rd = 0; rd < ROUNDS; ++rd) bsum[rd] = 0.0f;
-  auto store_loads = [&](const Staged& sg, bool have_g, int gbuf, int slot0, bool counted = true) {
+  auto store_loads = [&](Staged& sg, bool have_g, int gbuf, int slot0, bool counted = true) {
     uint32_t g_keep[4], x_keep[4];
     if (!ALLIN && sg.masked) {
+      if (__builtin_amdgcn_ballot_w64(sg.over != 0u) != 0) fetch_over(sg, have_g);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         g_keep[j] = (((sg.g_cols >> (2 * j)) & 1u) * 0xffffu) | (((sg.g_cols >> (2 * j + 1)) & 1u) * 0xffff0000u);
@@ -635,18 +634,12 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
       }
     }
   };
-  auto compute_group = [&](int gbuf, int base, int cgi) {
-    Frags f;
-    read_group(f, gbuf, base, cgi);
-    mfma_group(f);
-  };
-
   // Stage k of this workgroup reads ring rows base_k .. base_k + XR - 1 with base_k = NEW k mod RING: its
   // first OLD rows are the last ones the stage before read, its new rows go behind them. A stage that does
   // not continue the strip of the stage before fetches the old rows itself, into those same ring rows (as
   // many rows as the new ones at stride 2, of which the last is the old one: the others go to ring rows
   // that nobody reads).
-  static_assert(GROUPS == 2 || (GROUPS == 1 && !ALLIN), "the stage loop is written for one or two column groups per wavefront");
+  static_assert(GROUPS == 2 || GROUPS == 1, "the stage loop is written for one or two column groups per wavefront");
   auto wrap = [](int v) { return v >= RING ? v - RING : v; };
   if (s_begin < s_end) {
     Staged stg;
@@ -657,7 +650,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     store_loads(stg, true, 0, OLD);
     issue_loads(stg, c_next, false, 0);
     store_loads(stg, false, 0, (OLD - NEW + RING) % RING);
-    if constexpr (ALLIN) {
+    {
       // The loads of a stage are issued, and the registers of the stage before stored, in EVERY
       // stage: the cursor stops at the workgroup's last stage, which the last two stages fetch
       // again for nothing, and what the last stage stores nobody reads. A load or a store under
@@ -681,21 +674,22 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
       const bool stage_first = CWAVES == 8 && (wave & 4) != 0;
       for (long long st = s_begin; st < s_end; ++st) {
         Frags f0, f1;
+        (void)f1;
         if (stage_first) {
           store_loads(stg, true, gbuf ^ 1, wrap(base + XR), st + 1 < s_end);
           issue_loads(stg, c_next, true, 1);
         }
         if (wave < CWAVES) {
           read_group(f0, gbuf, base, 0);
-          read_group(f1, gbuf, base, 1);
+          if (GROUPS == 2) read_group(f1, gbuf, base, 1);
           mfma_group(f0);
-          if (CWAVES == 8) mfma_group(f1);
+          if (GROUPS == 2 && CWAVES == 8) mfma_group(f1);
         }
         if (!stage_first) {
           store_loads(stg, true, gbuf ^ 1, wrap(base + XR), st + 1 < s_end);
           issue_loads(stg, c_next, true, 1);
         }
-        if (CWAVES != 8 && wave < CWAVES) mfma_group(f1);
+        if (GROUPS == 2 && CWAVES != 8 && wave < CWAVES) mfma_group(f1);
         if (st + 3 < s_end) advance(c_next);
         __syncthreads();
         if (st + 1 < s_end && c_store.hp == 0) {
@@ -707,34 +701,6 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
           // the compiler cannot see a load waited for on every path, it waits at the loop's end,
           // and that wait takes the stage's own loads with it. vmcnt(0), said once, here:
           __builtin_amdgcn_s_waitcnt(0x0F70);
-          __syncthreads();
-        }
-        advance(c_store);
-        base = wrap(base + NEW);
-        gbuf ^= 1;
-      }
-    } else {
-      advance(c_next);
-      Cursor c_store = c_next;          // stage whose registers are stored next (st + 1)
-      if (s_begin + 1 < s_end) {
-        issue_loads(stg, c_next, true, 1);
-        advance(c_next);
-      }
-      __syncthreads();
-      for (long long st = s_begin; st < s_end; ++st) {
-        if (wave < CWAVES) compute_group(gbuf, base, 0);
-        if (st + 1 < s_end) store_loads(stg, true, gbuf ^ 1, wrap(base + XR));
-        if (st + 2 < s_end) {
-          issue_loads(stg, c_next, true, 1);
-          advance(c_next);
-        }
-        if (GROUPS == 2 && wave < CWAVES) compute_group(gbuf, base, 1);
-        __syncthreads();
-        if (st + 1 < s_end && c_store.hp == 0) {
-          // the next stage starts a new strip: its first two x rows, on the spot
-          Staged top;
-          issue_loads(top, c_store, false, 0);
-          store_loads(top, false, 0, wrap(base + OLD));
           __syncthreads();
         }
         advance(c_store);
