@@ -432,7 +432,7 @@ struct TokenWalk {
 // brought there by direct transfers a stage ahead; the fragments, whose contraction runs over the tokens, come from
 // transposing LDS reads (ds_read_b64_tr_b16, as in the attention backward). Chunk c of a row sits at c ^ 4 (row % 4): the
 // four rows a transposing read of 16 lanes touches then cover all banks. No registers are staged and no vector
-// instruction transposes: with its reduction 92 us for 32768 tokens, 1536 x 512 (101 us with both), 1132 us for
+// instruction transposes: with its reduction 72 us for 32768 tokens, 1536 x 512 (101 us with both and a round more), 1132 us for
 // 8192 x 8192 x 8192 (1294). A batch entry may be of any length: the octet-wise staging took multiples of 8 tokens
 // only and left the rest to the FMA kernel (5 x 590 tokens, 896 features, qkv and output projection: 2247 -> 250 us). The bias gradient is one more matrix instruction with ones, in the first column of tiles.
 template <int IM, int JN, int WM, int WN>
@@ -446,7 +446,7 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   // Workgroups go to the 8 XCDs round-robin. The few tiles of 128 x 128 of a split are gathered on one XCD, where they
   // meet in its L2 (65536 tokens, 512 x 128: 26.6 us, 29.5 spread). The 256-wide ones, which stream twice as much
-  // per workgroup, are spread (32768 tokens, 1536 x 512: 92 us, 113 gathered).
+  // per workgroup, are spread (32768 tokens, 1536 x 512 in 22 splits: 92 us, 113 gathered).
   int id = blockIdx.x;
   if (T == 128) {
     const int per_xcd = gridDim.x / 8;
@@ -829,30 +829,48 @@ bool map_vec_ok(const Map& m, long long features) {
   if (features % 8 != 0) return false;
   return m.heads ? (m.D % 8 == 0) : (m.ld % 8 == 0);
 }
-// Token ranges (splits) the contraction is cut into so that `tiles` tiles fill the chip; a
-// split is worth its partial tile from about 8 stages on.
-int splits_for(long long rows, int tiles, int target, bool small_tiles = false) {
-  const long long stages = (rows + BR - 1) / BR;
-  long long want = (target + tiles - 1) / tiles;
-  // at most 64 splits, but with one to three 128-wide tiles as many as put a workgroup on every compute
-  // unit: a compute unit streams its operands at some 20 GB/s, so 64 workgroups leave three quarters of
-  // the memory system idle (128 x 128 over 65536 tokens: 23 -> 13 us, the reduction 5 -> 6 us)
-  const long long cap = !small_tiles || tiles * 64 >= 256 ? 64 : 256 / tiles;
-  if (want > stages / (cap > 64 ? 4 : 8)) want = stages / (cap > 64 ? 4 : 8);
+// Tile edge of the weight-gradient kernel: 256 (half the operand traffic per MFMA, one workgroup
+// per compute unit) when such tiles and their splits still fill most of the chip, else 128. A split (a range of
+// tokens) is worth its partial tile from about 8 stages on.
+constexpr int TN_MOST_SPLITS = 64;
+long long tn_stages(long long rows) { return (rows + BR - 1) / BR; }
+int tn_tile(long long rows, int n, int c) {
+  if (n < 256 || c < 256) return 128;
+  const long long tiles = (long long)jg::cdiv(n, 256) * jg::cdiv(c, 256);
+  const long long most = tn_stages(rows) / 8;
+  return tiles * (most < 1 ? 1 : most < TN_MOST_SPLITS ? most : TN_MOST_SPLITS) >= 192 ? 256 : 128;
+}
+// Token ranges the contraction is cut into so that the tiles fill the chip.
+int tn_splits(long long rows, int n, int c) {
+  const int t = tn_tile(rows, n, c);
+  const long long tiles = (long long)jg::cdiv(n, t) * jg::cdiv(c, t), stages = tn_stages(rows);
+  if (t == 256) {
+    // One workgroup fits a compute unit, so a few more than 256 of them cost a second round: 12 tiles in 22 splits
+    // (1536 x 512 over 32768 tokens) took 88 us, in 21 splits 72. The number of splits with the least of: rounds of
+    // 256 times the stages of a split (1.7 us each, 5 us around them), and the partials, written and read back at about
+    // 6 TB/s. 3072 x 1024 over 8192 tokens 102 -> 74 us (6 -> 5 splits), 2112 x 704 over 20000 125 -> 91 us (10 -> 9),
+    // 512 x 512 over 32768 44 -> 41 us (64 -> 47).
+    int best = 1;
+    double least = 0.0;
+    for (int k = 1; k <= TN_MOST_SPLITS && (k == 1 || k <= stages / 8); ++k) {
+      const double rounds = (double)((tiles * k + 255) / 256), walk = (double)((stages + k - 1) / k);
+      const double us = rounds * (walk * 1.7 + 5.0) + k * (double)n * c * 8.0 / 6.0e6;
+      if (k == 1 || us < least) {
+        least = us;
+        best = k;
+      }
+    }
+    return best;
+  }
+  // 128: two workgroups a compute unit, two rounds of them; at most 64 splits, but with one to three tiles as many
+  // as put a workgroup on every compute unit: a compute unit streams its operands at some 20 GB/s, so 64 workgroups
+  // leave three quarters of the memory system idle (128 x 128 over 65536 tokens: 23 -> 13 us, the reduction 5 -> 6 us)
+  const long long cap = tiles * TN_MOST_SPLITS >= 256 ? TN_MOST_SPLITS : 256 / tiles;
+  long long want = (1024 + tiles - 1) / tiles;
+  if (want > stages / (cap > TN_MOST_SPLITS ? 4 : 8)) want = stages / (cap > TN_MOST_SPLITS ? 4 : 8);
   if (want < 1) want = 1;
   if (want > cap) want = cap;
   return (int)want;
-}
-// Tile edge of the weight-gradient kernel: 256 (half the operand traffic per MFMA, one workgroup
-// per compute unit) when such tiles and their splits still fill most of the chip, else 128.
-int tn_tile(long long rows, int n, int c) {
-  if (n < 256 || c < 256) return 128;
-  const int tiles = jg::cdiv(n, 256) * jg::cdiv(c, 256);
-  return tiles * splits_for(rows, tiles, 256) >= 192 ? 256 : 128;
-}
-int tn_splits(long long rows, int n, int c) {
-  const int t = tn_tile(rows, n, c);
-  return splits_for(rows, jg::cdiv(n, t) * jg::cdiv(c, t), t == 256 ? 256 : 1024, t == 128);
 }
 
 template <int IM, int JN, int WM, int WN>
