@@ -179,7 +179,10 @@ def test_fp32_parameters_get_unrounded_fp32_gradients(shape, n_out, dev):
     assert rel_l2(wd.grad.cpu(), gw) < 1e-5 and rel_l2(bd.grad.cpu(), gb) < 1e-5
 
 
-@pytest.mark.parametrize("rows,dim,hid,with_res", [((3, 50), 64, 256, True), ((200,), 128, 512, True), ((2, 33), 40, 96, False)])
+@pytest.mark.parametrize("rows,dim,hid,with_res", [
+    ((3, 50), 64, 256, True), ((200,), 128, 512, True), ((2, 33), 40, 96, False),
+    ((33001,), 128, 520, True), ((9, 1001), 72, 264, True),  # 256- and 128-wide tiles that read ahead past the last token and feature
+])
 def test_gelu_mlp_fused_epilogues(rows, dim, hid, with_res, dev):
     """residual + Linear(GELU(Linear(x))) on the fused epilogues (GELU beside the pre-activation, the
     GELU derivative and the residual sum on the way out of a GEMM) against fp64 autograd of the same
