@@ -124,6 +124,13 @@ PRIM_CASES = [
     (2, 48, 32, (20, 22), (3, 3), (2, 2), (1, 1), (1, 1), 2),
     (1, 32, 64, (17, 19), (5, 5), (1, 1), (2, 2), (1, 1), 4),
     (1, 24, 24, (6, 10, 12), (3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 2, 2), 3),
+    # fp32: few channels or a few beyond a multiple of 16 (the part products of all blocks counted through); several
+    # tiles of produced channels that share the chip, with more and with fewer pixel tiles than it has compute units
+    (2, 3, 5, (40, 71), (3, 3), (1, 1), (1, 1), (1, 1)),
+    (1, 17, 33, (19, 66), (3, 3), (1, 1), (1, 1), (1, 1)),
+    (2, 5, 65, (36, 70), (3, 3), (2, 2), (1, 1), (1, 1)),
+    (1, 4, 8, (5, 18, 20), (3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1)),
+    (3, 8, 160, (129, 200), (3, 3), (1, 1), (1, 1), (1, 1)),
 ]
 
 
