@@ -379,12 +379,8 @@ int launch_nt(NtParams& p, hipStream_t s, const char* who) {
   JG_REQUIRE(tiles < (1ll << 30), "%s: too many tiles", who);
   p.tiles = (int)tiles;
   void (*kern)(NtParams) = &proj_nt_kernel<IM, JN, WM, WN>;
-  static bool reserved = false;
-  if (!reserved) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS) != hipSuccess)
-      JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, SH::LDS);
-    reserved = true;
-  }
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS) != hipSuccess)
+    JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, SH::LDS);
   // as many workgroups as fit at once (a multiple of 8: one share per XCD)
   const long long fit = 256 * (160 * 1024 / SH::LDS);
   const unsigned grid = (unsigned)(((tiles < fit ? tiles : fit) + 7) / 8 * 8);
@@ -895,12 +891,8 @@ int launch_tn(TnParams& p, int splits, hipStream_t s, const char* who) {
   p.tiles_c = jg::cdiv(p.C, SH::T);
   p.tiles = jg::cdiv(p.N, SH::T) * p.tiles_c;
   void (*kern)(TnParams) = &proj_tn_kernel<IM, JN, WM, WN>;
-  static bool reserved = false;
-  if (!reserved) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS) != hipSuccess)
-      JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, SH::LDS);
-    reserved = true;
-  }
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS) != hipSuccess)
+    JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, SH::LDS);
   kern<<<(unsigned)p.tiles * (unsigned)splits, SH::THREADS, SH::LDS, s>>>(p);
   JG_CHECK_LAUNCH(who);
   return JG_OK;
