@@ -823,7 +823,7 @@ __global__ __launch_bounds__(256) void fold_rows_kernel(Table tab,
   const T* orow = own + ((p * Da + (d + g.lo[0])) * Ha + (h + g.lo[1])) * (long long)Wa + g.lo[2];
   T* drow = dst + (long long)row * W;
   // defer_border: such a row only gets `0 + own` here, like the columns of a plain row that no
-  // neighbour reaches, and fold_border_rows_kernel sums it in full afterwards, a whole wavefront
+  // neighbour reaches, and fold_border_kernel sums it in full afterwards, a whole wavefront
   // per row (in a volume every eighth wavefront of this kernel holds such a row and would walk
   // the long path with a few lanes active).
   if (!row_plain && !defer_border) {
@@ -945,12 +945,14 @@ __global__ __launch_bounds__(256) void fold_rows_kernel(Table tab,
 
 
 // In-place second half of a fold: gx already holds `0 + own`; only the cells that a
-// neighbour reaches change. Two kernels: the rows that a D or H neighbour reaches are
-// summed in full, one wavefront per row; of the other rows only the first and last
-// columns change, one lane per cell.
+// neighbour reaches change. The rows that a D or H neighbour reaches are summed in full,
+// up to a wavefront per row; of the other rows only the first and last columns change, one lane
+// per cell. Both in one launch, the blocks of the rows first: they are few and wait for chains of
+// loads, the columns' blocks for a cache line per cell, and neither fills the chip (8 x 64
+// channels of 1024 x 1024: 66 -> 55 us, 2 x 32 of 128 x 128 x 128 87 -> 72 us; two launches before).
 struct BorderPlan {
   uint32_t rows_per_plane;  // rows of a plane that a D or H neighbour reaches
-  uint32_t total;           // work items of the launch
+  uint32_t row_items, col_items, row_blocks;  // such rows, edge cells of all rows; blocks that take rows
   int nbd, nbh;             // border depths / border rows of a non-border depth
   int n_edge, head;         // W-edge cells of a row: columns [0, head) and [W - lo, W)
   int lpr;                  // lanes per row of the rows kernel
@@ -959,13 +961,12 @@ struct BorderPlan {
 
 
 template <int DT>
-__global__ __launch_bounds__(256) void fold_border_rows_kernel(Table tab, typename Arith<DT>::T* __restrict__ gx,
-                                                               Geom g, BorderPlan bp) {
+__device__ __forceinline__ void fold_border_rows(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp) {
   typedef typename Arith<DT>::T T;
   constexpr int V = Bits<T>::V;
   // a row is owned by bp.lpr lanes (a power of two up to 64: a whole wavefront for long rows)
   const uint32_t item = (blockIdx.x * 256u + threadIdx.x) / (uint32_t)bp.lpr;
-  if (item >= bp.total) return;
+  if (item >= bp.row_items) return;
   const int lane = threadIdx.x & (bp.lpr - 1);
   const int D = g.n[0], H = g.n[1], W = g.n[2];
   const uint32_t pp = mdiv(item, bp.div_rows);
@@ -989,11 +990,10 @@ __global__ __launch_bounds__(256) void fold_border_rows_kernel(Table tab, typena
 }
 
 template <int DT>
-__global__ __launch_bounds__(256) void fold_border_cols_kernel(Table tab, typename Arith<DT>::T* __restrict__ gx,
-                                                               Geom g, BorderPlan bp) {
+__device__ __forceinline__ void fold_border_cols(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp) {
   typedef typename Arith<DT>::T T;
-  const uint32_t item = blockIdx.x * 256u + threadIdx.x;  // (row, edge cell), cell fastest
-  if (item >= bp.total) return;
+  const uint32_t item = (blockIdx.x - bp.row_blocks) * 256u + threadIdx.x;  // (row, edge cell), cell fastest
+  if (item >= bp.col_items) return;
   const int D = g.n[0], H = g.n[1], W = g.n[2];
   const uint32_t row = mdiv(item, bp.div_edge);
   const int q = (int)(item - row * (uint32_t)bp.n_edge);
@@ -1018,6 +1018,13 @@ __global__ __launch_bounds__(256) void fold_border_cols_kernel(Table tab, typena
       acc = Arith<DT>::up(Arith<DT>::down(acc + Arith<DT>::up(s_hi[(long long)row * g.lo[2] + (c - up0)])));
   }
   *cell = Arith<DT>::down(acc);
+}
+
+// tab comes first among the parameters: its entries are read from the kernel-argument segment
+template <int DT>
+__global__ __launch_bounds__(256) void fold_border_kernel(Table tab, typename Arith<DT>::T* __restrict__ gx, Geom g, BorderPlan bp) {
+  if (blockIdx.x < bp.row_blocks) fold_border_rows<DT>(gx, g, bp);
+  else fold_border_cols<DT>(gx, g, bp);
 }
 
 Magic make_magic(uint32_t d) {
@@ -1368,16 +1375,20 @@ bool border_plan(const Geom& g, BorderPlan* bp, unsigned long long* row_items, u
 }
 // The rows a D or H neighbour reaches, summed in full in place; false if there are too many.
 template <int DT>
-bool launch_border_rows(const Table& tab, void* gx, const Geom& g, BorderPlan bp, unsigned long long row_items, hipStream_t s) {
+bool launch_border(const Table& tab, void* gx, const Geom& g, BorderPlan bp, unsigned long long row_items,
+                   unsigned long long col_items, hipStream_t s) {
   typedef typename Arith<DT>::T T;
-  if (row_items == 0) return true;
-  bp.total = (uint32_t)row_items;
   const int vecs = g.n[2] / (16 / (int)sizeof(T));
   bp.lpr = 1;
   while (bp.lpr < 64 && bp.lpr < vecs) bp.lpr *= 2;
   const unsigned long long threads = row_items * (unsigned long long)bp.lpr;
-  if (threads >= (1ull << 32)) return false;
-  fold_border_rows_kernel<DT><<<(unsigned)((threads + 255) / 256), 256, 0, s>>>(tab, static_cast<T*>(gx), g, bp);
+  if (threads >= (1ull << 32) || col_items >= (1ull << 32)) return false;
+  bp.row_items = (uint32_t)row_items;
+  bp.col_items = (uint32_t)col_items;
+  bp.row_blocks = (uint32_t)((threads + 255) / 256);
+  const unsigned long long blocks = bp.row_blocks + (col_items + 255) / 256;
+  if (blocks == 0) return true;
+  fold_border_kernel<DT><<<(unsigned)blocks, 256, 0, s>>>(tab, static_cast<T*>(gx), g, bp);
   return true;
 }
 }  // namespace
@@ -1426,13 +1437,13 @@ extern "C" int jg_halo_fold_3d(void* gx, const void* gx_aug, const void* const s
     bool ok = true;
     if (dtype == JG_F32) {
       fold_rows_kernel<JG_F32><<<blocks, 256, 0, s>>>(tab, static_cast<uint32_t*>(gx), static_cast<const uint32_t*>(gx_aug), g, pl, defer);
-      if (defer) ok = launch_border_rows<JG_F32>(tab, gx, g, bp, row_items, s);
+      if (defer) ok = launch_border<JG_F32>(tab, gx, g, bp, row_items, 0, s);
     } else if (dtype == JG_BF16) {
       fold_rows_kernel<JG_BF16><<<blocks, 256, 0, s>>>(tab, static_cast<uint16_t*>(gx), static_cast<const uint16_t*>(gx_aug), g, pl, defer);
-      if (defer) ok = launch_border_rows<JG_BF16>(tab, gx, g, bp, row_items, s);
+      if (defer) ok = launch_border<JG_BF16>(tab, gx, g, bp, row_items, 0, s);
     } else {
       fold_rows_kernel<JG_F16><<<blocks, 256, 0, s>>>(tab, static_cast<uint16_t*>(gx), static_cast<const uint16_t*>(gx_aug), g, pl, defer);
-      if (defer) ok = launch_border_rows<JG_F16>(tab, gx, g, bp, row_items, s);
+      if (defer) ok = launch_border<JG_F16>(tab, gx, g, bp, row_items, 0, s);
     }
     JG_REQUIRE(ok, "jg_halo_fold_3d: too many border rows");
     JG_CHECK_LAUNCH("jg_halo_fold_3d");
@@ -1482,16 +1493,9 @@ extern "C" int jg_halo_fold_border_3d(void* gx, const void* const strips[27],
   BorderPlan bp;
   unsigned long long row_items = 0, col_items = 0;
   JG_REQUIRE(border_plan(g, &bp, &row_items, &col_items), "jg_halo_fold_border_3d: too many rows (%llu)", nrows);
-#define JG_BORDER(DT)                                                                                   \
-  do {                                                                                                  \
-    typedef Arith<DT>::T T;                                                                             \
-    JG_REQUIRE(launch_border_rows<DT>(tab, gx, g, bp, row_items, s),                                    \
-               "jg_halo_fold_border_3d: too many border rows (%llu)", row_items);                      \
-    if (col_items > 0) {                                                                                \
-      bp.total = (uint32_t)col_items;                                                                   \
-      fold_border_cols_kernel<DT><<<(unsigned)((col_items + 255) / 256), 256, 0, s>>>(tab, static_cast<T*>(gx), g, bp); \
-    }                                                                                                   \
-  } while (0)
+#define JG_BORDER(DT)                                                  \
+  JG_REQUIRE(launch_border<DT>(tab, gx, g, bp, row_items, col_items, s), \
+             "jg_halo_fold_border_3d: too many border rows (%llu)", row_items)
   if (dtype == JG_F32) JG_BORDER(JG_F32);
   else if (dtype == JG_BF16) JG_BORDER(JG_BF16);
   else JG_BORDER(JG_F16);
