@@ -427,6 +427,10 @@ int jg_proj_nt_fused_heads(void* out, void* aux, int epilogue, const void* a, co
 int jg_cast_params(void* const* dst, void* const* dst_t, const void* const* src, const int32_t* rows, const int32_t* cols,
                    int n, void* stream);
 
+/* dst (cols, rows) = the transpose of src (rows, cols), contiguous matrices of 16-bit values; both sizes multiples of
+ * 8 and both pointers 16-byte aligned, else JG_ERR_UNSUPPORTED. dst and src do not overlap. */
+int jg_transpose16(void* dst, const void* src, int64_t rows, int64_t cols, void* stream);
+
 /* gw[n][c] = sum_r g(r, n) * x(r, c)  (n, c) row-major, and gb[n] = sum_r g(r, n)
  * (gb may be NULL): weight and bias gradient of a projection (torch's
  * Linear backward; g = grad of the projection's output, x = its input).

@@ -223,6 +223,7 @@ SIGNATURES: dict[str, tuple] = {
         c_int,
         [POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p), POINTER(c_int32), POINTER(c_int32), c_int, c_void_p],
     ),
+    "jg_transpose16": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
     "jg_proj_nt": (
         c_int,
         [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int,

@@ -820,6 +820,31 @@ __global__ __launch_bounds__(256) void cast_params_kernel(CastArgs a) {
     if (c0 + i < cols && r0 + x < rows) a.dst_t[m][(size_t)(c0 + i) * rows + r0 + x] = tile[x][i];
 }
 
+// dst (cols, rows) = src (rows, cols)^T, 16-bit values, both sizes multiples of 8: a 64 x 64 tile per block, 16-byte
+// pieces both ways, turned on the way into LDS. What a weight of some MB waits for is one memory latency and the
+// launch: 1536 x 512 7.3 us with torch's copy, 3.4 here; 512 x 512 5.6 and 3.4.
+__global__ __launch_bounds__(256) void transpose16_kernel(uint16_t* __restrict__ dst, const uint16_t* __restrict__ src,
+                                                          long long rows, long long cols, int tiles_c) {
+  __shared__ __attribute__((aligned(16))) uint16_t tile[64][72];
+  const long long r0 = (long long)(blockIdx.x / tiles_c) * 64, c0 = (long long)(blockIdx.x % tiles_c) * 64;
+  const int piece = threadIdx.x & 7, line = threadIdx.x >> 3;  // 8 values, and the row (or column) they are of
+#pragma unroll
+  for (int i = 0; i < 64; i += 32) {
+    const long long r = r0 + line + i, c = c0 + piece * 8;
+    if (r < rows && c < cols) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(src + r * cols + c);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) tile[piece * 8 + e][line + i] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 64; i += 32) {
+    const long long c = c0 + line + i, r = r0 + piece * 8;
+    if (c < cols && r < rows) *reinterpret_cast<u32x4*>(dst + c * rows + r) = *reinterpret_cast<const u32x4*>(&tile[line + i][piece * 8]);
+  }
+}
+
 // --------------------------------------------------------------------- host
 int make_map(Map* m, int heads, long long features, long long rows, int B, int H, int S, int D, const char* who,
              const char* what) {
@@ -1002,6 +1027,21 @@ int jg_cast_params(void* const* dst, void* const* dst_t, const void* const* src,
   }
   if (blocks == 0) return JG_OK;
   cast_params_kernel<<<(unsigned)blocks, 256, 0, static_cast<hipStream_t>(stream)>>>(a);
+  JG_CHECK_LAUNCH(who);
+  return JG_OK;
+}
+
+int jg_transpose16(void* dst, const void* src, int64_t rows, int64_t cols, void* stream) {
+  const char* who = "jg_transpose16";
+  JG_REQUIRE(rows >= 0 && cols >= 0, "%s: bad sizes rows=%lld cols=%lld", who, (long long)rows, (long long)cols);
+  if (rows == 0 || cols == 0) return JG_OK;
+  JG_REQUIRE(dst && src, "%s: null pointer", who);
+  if (rows % 8 != 0 || cols % 8 != 0 || !aligned16(dst) || !aligned16(src))
+    JG_FAIL(JG_ERR_UNSUPPORTED, "%s: sizes that are multiples of 8 and 16-byte aligned matrices only", who);
+  const long long tiles_r = (rows + 63) / 64, tiles_c = (cols + 63) / 64;
+  JG_REQUIRE(tiles_r < (1ll << 31) / tiles_c, "%s: too large", who);
+  transpose16_kernel<<<(unsigned)(tiles_r * tiles_c), 256, 0, static_cast<hipStream_t>(stream)>>>(
+      static_cast<uint16_t*>(dst), static_cast<const uint16_t*>(src), rows, cols, (int)tiles_c);
   JG_CHECK_LAUNCH(who);
   return JG_OK;
 }

@@ -140,6 +140,17 @@ def cast_parameters(weights, biases) -> tuple:
     return w, wt, b
 
 
+def _transpose(w: torch.Tensor) -> torch.Tensor:
+    """Contiguous transpose of a matrix."""
+    n, k = w.shape
+    if not (w.is_cuda and w.itemsize == 2 and w.is_contiguous() and n % 8 == 0 and k % 8 == 0 and w.data_ptr() % 16 == 0):
+        return w.t().contiguous()
+    out = torch.empty(k, n, dtype=w.dtype, device=w.device)
+    lib = _lib.load()
+    _lib.check(lib.jg_transpose16(_lib.ptr(out), _lib.ptr(w), n, k, _lib.stream_ptr(w.device)), "jg_transpose16")
+    return out
+
+
 def _transposed(ctx, w: torch.Tensor) -> torch.Tensor:
     """The transposed weight of the input-gradient GEMM: what came with the cast (:func:`cast_parameters`), the
     remembered copy of the parameter when casts are remembered and the parameter is still the one the forward
@@ -149,7 +160,7 @@ def _transposed(ctx, w: torch.Tensor) -> torch.Tensor:
     ref = getattr(ctx, "weight_ref", None)
     if _remember_casts and ref is not None and ref._version == ctx.weight_version:
         return _cast_cached(ref, w.dtype, transposed=True)
-    return w.t().contiguous()
+    return _transpose(w)
 
 
 def _grad_dtype(compute: torch.dtype, dtypes) -> torch.dtype:
@@ -393,7 +404,7 @@ class _GeluMlp(torch.autograd.Function):
             if getattr(ctx, "weights_t", None) is not None:
                 return ctx.weights_t[i]
             ref, version = ctx.refs[i]
-            return _cast_cached(ref, wc.dtype, transposed=True) if _remember_casts and ref._version == version else wc.t().contiguous()
+            return _cast_cached(ref, wc.dtype, transposed=True) if _remember_casts and ref._version == version else _transpose(wc)
 
         gw2, gb2 = _tn(g, act, rows, n_out, hid, False, False, (1, 1, 1, 1), dt_b2 is not None,
                        _grad_dtype(g.dtype, (dt_w2, dt_b2)))

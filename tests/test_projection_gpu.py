@@ -258,6 +258,18 @@ def test_fused_projection_entry_refuses_what_it_has_no_kernel_for(dev):
     assert rel_l2(y, ref) < 1e-5
 
 
+@pytest.mark.parametrize("n,k,dtype", [
+    (8, 8, torch.bfloat16), (64, 72, torch.bfloat16), (1536, 520, torch.float16), (200, 8, torch.bfloat16), (7, 16, torch.bfloat16), (16, 24, torch.float32),
+], ids=str)
+def test_transpose_is_exact(n, k, dtype, dev):
+    """Edges of the 64 x 64 tiles, sizes and types that torch's copy takes, and a matrix off the 16-byte grid."""
+    w = torch.randn(n * k + 8, device=dev).to(dtype)
+    for at in (0, 1):
+        m = w[at:at + n * k].view(n, k)
+        got = jp._transpose(m)
+        assert got.is_contiguous() and torch.equal(got, m.t())
+
+
 @pytest.mark.parametrize("b,s,c,n_out,heads", [
     (1, 1, 8, 24, 1), (3, 5, 64, 192, 2), (2, 63, 72, 200, 1), (5, 117, 136, 264, 3), (1, 65, 64, 64, 2), (7, 129, 256, 512, 4),
     (2, 4100, 512, 1536, 8), (9, 1001, 264, 768, 4),
