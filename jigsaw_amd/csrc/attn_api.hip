@@ -57,7 +57,7 @@ int check_shape(const char* who, int64_t batch, int64_t sq, int64_t sk, int64_t 
   return JG_OK;
 }
 
-// The window kernels move 16 bytes per lane.
+// Every kernel but the one-thread-per-row ones moves 16 bytes per lane.
 bool aligned16(std::initializer_list<const void*> ptrs) {
   for (const void* q : ptrs)
     if ((reinterpret_cast<uintptr_t>(q) & 15) != 0) return false;
@@ -97,7 +97,8 @@ extern "C" int jg_attn_fwd(void* out, float* lse, const void* q, const void* k, 
   JG_REQUIRE(bias == nullptr || bias_period >= 1, "%s: bias_period must be >= 1", who);
   if (batch == 0 || sq == 0) return JG_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (jg::attn_mfma_fwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr))
+  if (jg::attn_mfma_fwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr) &&
+      aligned16({out, q, k, v, out_acc}))
     return jg::attn_mfma_fwd_chunks(out, lse, q, &k, &v, 1, batch, (int)sq, (int)sk, scale, out_acc, lse_acc, s);
   if (out_acc == nullptr && jg::attn_window_supported(batch, (int)sq, (int)sk, (int)d, dtype) &&
       aligned16({out, q, k, v, bias}))
@@ -145,7 +146,8 @@ extern "C" int jg_attn_bwd(void* dq, void* dk, void* dv, const void* dout, const
     JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, workspace_bytes,
             jg_attn_bwd_workspace_bytes(batch, sq, sk, d));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dbias == nullptr && jg::attn_mfma_bwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr))
+  if (dbias == nullptr && jg::attn_mfma_bwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr) &&
+      aligned16({dq, dk, dv, dout, q, k, v, out}))
     return jg::attn_mfma_bwd_chunks(dq, &dk, &dv, dout, q, &k, &v, 1, out, lse, batch, (int)sq, (int)sk, scale,
                                     workspace, s);
   if (jg::attn_window_supported(batch, (int)sq, (int)sk, (int)d, dtype) &&
@@ -180,10 +182,10 @@ extern "C" int jg_attn_fwd_chunks(void* out, float* lse, const void* q, const vo
   if (rc) return rc;
   if (batch == 0 || sq == 0) return JG_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (jg::attn_mfma_fwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, false))
+  const bool aligned = aligned16({out, q}) && chunks_aligned16(n_chunks, {k, v});
+  if (aligned && jg::attn_mfma_fwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, false))
     return jg::attn_mfma_fwd_chunks(out, lse, q, k, v, (int)n_chunks, batch, (int)sq, (int)sk, scale, nullptr, nullptr, s);
-  if (jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, false) && aligned16({out, q}) &&
-      chunks_aligned16(n_chunks, {k, v}))
+  if (aligned && jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, false))
     return jg::attn_wide_fwd_chunks(out, lse, q, k, v, (int)n_chunks, batch, (int)sq, (int)sk, (int)d, dtype, scale,
                                     nullptr, nullptr, s);
   JG_FAIL(JG_ERR_UNSUPPORTED, "%s: bf16 or fp16, d a multiple of 8 up to 128, 16-byte aligned tensors", who);
@@ -205,11 +207,11 @@ extern "C" int jg_attn_bwd_chunks(void* dq, void* const* dk, void* const* dv, co
     JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, workspace_bytes,
             jg_attn_bwd_workspace_bytes(batch, sq, sk, d));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (jg::attn_mfma_bwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, false))
+  const bool aligned = aligned16({dq, dout, q, out}) && chunks_aligned16(n_chunks, {k, v, dk, dv});
+  if (aligned && jg::attn_mfma_bwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, false))
     return jg::attn_mfma_bwd_chunks(dq, dk, dv, dout, q, k, v, (int)n_chunks, out, lse, batch, (int)sq, (int)sk, scale,
                                     workspace, s);
-  if (jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, false) && aligned16({dq, dout, q, out}) &&
-      chunks_aligned16(n_chunks, {k, v, dk, dv}))
+  if (aligned && jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, false))
     return jg::attn_wide_bwd_chunks(dq, dk, dv, dout, q, k, v, (int)n_chunks, out, lse, batch, (int)sq, (int)sk, (int)d,
                                     dtype, scale, workspace, s);
   JG_FAIL(JG_ERR_UNSUPPORTED, "%s: bf16 or fp16, d a multiple of 8 up to 128, 16-byte aligned tensors", who);

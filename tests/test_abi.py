@@ -5,6 +5,7 @@ import re
 from pathlib import Path
 
 import pytest
+import torch
 
 import jigsaw_amd
 from jigsaw_amd import _lib
@@ -59,3 +60,22 @@ def test_bad_arguments_are_rejected_without_a_gpu():
     assert b"wider than the tile" in lib.jg_last_error()
     with pytest.raises(ValueError):
         _lib.check(rc, "jg_halo_assemble_3d")
+
+
+@pytest.mark.parametrize("d", [64, 96])
+@pytest.mark.parametrize("which", ["q", "out", "k", "dk"])
+def test_misaligned_chunks_are_refused_without_a_gpu(which, d):
+    """jg_attn_fwd_chunks / jg_attn_bwd_chunks move 16 bytes per lane: a tensor that starts off a 16-byte boundary is
+    JG_ERR_UNSUPPORTED before anything is launched, at any length and head size."""
+    lib = jigsaw_amd.load()
+    at = {n: 0x1000 * (i + 1) + (2 if n == which else 0) for i, n in enumerate(("q", "out", "k", "v", "dq", "dk", "dv", "dout", "lse", "ws"))}
+    p = {n: ctypes.c_void_p(v) for n, v in at.items()}
+    one = lambda n: (ctypes.c_void_p * 1)(at[n])  # noqa: E731
+    bf16 = _lib.dtype_code(torch.bfloat16)
+    for sq, sk in ((100, 1000), (256, 128)):
+        if which != "dk":
+            rc = lib.jg_attn_fwd_chunks(p["out"], p["lse"], p["q"], one("k"), one("v"), 1, 2, sq, sk, d, 0.125, bf16, None)
+            assert rc == -2 and b"aligned" in lib.jg_last_error()
+        rc = lib.jg_attn_bwd_chunks(p["dq"], one("dk"), one("dv"), p["dout"], p["q"], one("k"), one("v"), 1, p["out"], p["lse"], 2,
+                                    sq, sk, d, 0.125, bf16, p["ws"], 1 << 20, None)
+        assert rc == -2 and b"aligned" in lib.jg_last_error()
