@@ -563,6 +563,9 @@ int jg_bias_grad(void* gb, const void* g, int64_t batch, int64_t channels,
  * q (batch, sq, d), k / v (batch, sk, d), dense, `batch` = all leading axes
  * flattened (b*h for the "bhsd" layout of jigsaw's sdpa / math cores). One dtype
  * per call; softmax and accumulation in fp32. Non-causal, no dropout.
+ * 16-bit calls without a bias round probabilities (and dS) to 16 bits before their second matrix product where the
+ * range of keys is long. Ranges (chunks) of fewer than 128 keys keep them in fp32, forward and backward; so do, in the
+ * forward at head sizes 96, 128 and bf16 64, the keys behind the last multiple of 128.
  * `bias` (optional, fp32): additive score bias / mask of shape
  * (bias_period, sq, sk); batch entry i uses bias[i % bias_period]
  * (windowed attention with a relative-position bias, examples/swin.py:146-151).

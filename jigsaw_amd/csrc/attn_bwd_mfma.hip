@@ -576,8 +576,9 @@ __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void at
 
 namespace jg {
 
+// (shorter chunks keep P and dS in fp32: attn_wide.hip)
 bool attn_mfma_bwd_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias) {
-  return dtype == JG_BF16 && !has_bias && d == D && sq > 0 && sk > 0 && sq <= ATTN_MAX_KEYS && sk <= ATTN_MAX_KEYS &&
+  return dtype == JG_BF16 && !has_bias && d == D && sq > 0 && sk >= EXACT_KEYS && sq <= ATTN_MAX_KEYS && sk <= ATTN_MAX_KEYS &&
          batch > 0 && batch <= 65535;
 }
 

@@ -38,6 +38,48 @@ inline ChunkTable chunk_table(const void* const* k, const void* const* v, void* 
   return tab;
 }
 
+// Which keys keep their probabilities in fp32. The kernels round P (and dS) to the 16 bits of the operands before P V
+// (dS K, dS^T Q, P^T dO) where a chunk is long. Of a chunk with fewer than EXACT_KEYS keys nothing is rounded, forward
+// and backward, nor are, in the forward, the keys behind the last multiple of EXACT_KEYS where the head fills a
+// kernel's width: there the values go into the matrix product as three bf16 parts (see parts8).
+constexpr int EXACT_KEYS = 128;
+inline int exact_from(int sk, int d, int dtype) {  // first key of a chunk whose probabilities the forward keeps in fp32
+  if (sk < EXACT_KEYS) return 0;
+  return d == 96 || d == 128 || (d == 64 && dtype == JG_BF16) ? sk / EXACT_KEYS * EXACT_KEYS : sk;
+}
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+// Eight fp32 values as three bf16 ones each that add up to them exactly: the upper 16 bits, those of the rest, and those
+// of what is left then (24 bits of significand in three pieces of 8, cut and not rounded, so that all three have
+// the value's sign). The products with bf16 operands are exact in the matrix cores' fp32 accumulators, so a
+// contraction over the parts is as exact as one in fp32, at three times the instructions and a fifth of the time of
+// the fp32 matrix instructions. An infinite value is its first part. POSITIVE (probabilities): the
+// lower parts are never 0, so that a probability that is not 0 times an infinite operand stays infinite as it does in fp32.
+template <bool POSITIVE>
+__device__ __forceinline__ void parts8(const float* v, bf16x8_t (&part)[3]) {
+  u32x4_t w[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = v[2 * i], b = v[2 * i + 1];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
+      w[t][i] = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
+      const float ha = __uint_as_float(ua & 0xffff0000u), hb = __uint_as_float(ub & 0xffff0000u);
+      a = a == ha ? 0.0f : a - ha;
+      b = b == hb ? 0.0f : b - hb;
+      if (POSITIVE) {
+        a = fmaxf(a, 1.1754943508222875e-38f);
+        b = fmaxf(b, 1.1754943508222875e-38f);
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 3; ++t) part[t] = __builtin_bit_cast(bf16x8_t, w[t]);
+}
+
 // Workgroup -> (batch entry, chunk, row block) of a grid (row blocks, batch entries, chunks). Consecutive
 // workgroup ids go to the 8 XCDs in turn; each XCD is given a contiguous range of the flat order (batch entry,
 // chunk, block), so the workgroups that stream the same K / V (or Q / dO) share one L2 instead of every L2

@@ -51,6 +51,7 @@ using jg::BlockOf;
 using jg::ChunkTable;
 using jg::block_of;
 using jg::chunk_entry;
+using jg::parts8;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -108,11 +109,13 @@ __device__ __forceinline__ void pair32(float v, float& a, float& b) {
   b = __uint_as_float(sw[1]);
 }
 
-// RAGGED: sq or sk is no multiple of 128. The same kernel with the key rows of a transfer clamped to the chunk's
-// last one (three vector instructions per transfer), the scores of keys past the end set to -inf, query rows
-// clamped when read and dropped when written. 24 heads x 1000 queries x 2 chunks of 1000 keys: 93 us forward + backward
-// of the ring, against 832 us when the lengths were brought to multiples of 128 on the host (copies, a remainder of 104
-// keys on the one-thread-per-row kernel, two merges). The aligned kernel keeps its transfers free of vector instructions.
+// RAGGED: sq or sk is no multiple of 128. Query rows are clamped when read and dropped when written, and the keys of a
+// chunk behind its last multiple of 128 go through a loop of their own after the pipeline, a tile per key quarter and
+// chunk: their probabilities are not rounded to 16 bits (see parts8), which a chunk shorter than 128 keys is all of. Key
+// rows past the chunk's end are clamped to the last one on the way in, cleared in V, and their scores set to -inf.
+// 24 heads x 1000 queries x 2 chunks of 1000 keys: 28.6 us (28.1 with the last keys in the pipeline and rounded), 8 chunks
+// 84.7 (80.2), 64 heads x 300 x 8 chunks of 300 39.2 (40.5); the ring of the first, forward and backward, 93 us, against
+// 832 when the lengths were brought to multiples of 128 on the host. The aligned kernel is not touched by any of it.
 template <bool RAGGED>
 __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdArgs p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -125,7 +128,8 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
   const int q0 = where.blk * BM + qg * 64;
   // every chunk is cut in four key quarters (one per pair of wavefronts); a quarter's tiles of all chunks
   // form one stream of ntiles tiles
-  const int qtiles = (p.sk + NQ * BN - 1) / (NQ * BN);
+  // (the whole tiles of a quarter: RAGGED leaves up to 127 keys of a chunk to the loop behind the pipeline)
+  const int qtiles = p.sk / (NQ * BN);
   const int ntiles = qtiles * p.nchunks;
   const float c2 = p.scale * 1.4426950408889634f;  // scores are handled in base 2
 
@@ -169,21 +173,11 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
   const char* vdma = chunk_entry(1, 0) + chunk_off;
   auto dma_tile = [&](int buf) {
     const uint32_t dst = lds_dma + (uint32_t)(buf * TILE_BYTES);
-    const int row = row_first + ld_tile * BN;
-    if (RAGGED) {
-      const uint32_t o0 = (uint32_t)min(row + (lane >> 3), p.sk - 1) * ROWB + dma_swz;
-      const uint32_t o1 = (uint32_t)min(row + 8 + (lane >> 3), p.sk - 1) * ROWB + dma_swz;
-      dma_1k(kdma, o0, dst);
-      dma_1k(kdma, o1, dst + 8 * ROWB);
-      dma_1k(vdma, o0, dst + KV_BYTES);
-      dma_1k(vdma, o1, dst + KV_BYTES + 8 * ROWB);
-    } else {
-      const long long off = (long long)row * ROWB;
-      dma_1k(kdma + off, dma_off, dst);
-      dma_1k(kdma + off + 8 * ROWB, dma_off, dst + 8 * ROWB);
-      dma_1k(vdma + off, dma_off, dst + KV_BYTES);
-      dma_1k(vdma + off + 8 * ROWB, dma_off, dst + KV_BYTES + 8 * ROWB);
-    }
+    const long long off = (long long)(row_first + ld_tile * BN) * ROWB;
+    dma_1k(kdma + off, dma_off, dst);
+    dma_1k(kdma + off + 8 * ROWB, dma_off, dst + 8 * ROWB);
+    dma_1k(vdma + off, dma_off, dst + KV_BYTES);
+    dma_1k(vdma + off + 8 * ROWB, dma_off, dst + KV_BYTES + 8 * ROWB);
     if (ld_left > 0) {
       --ld_left;
       if (++ld_tile == qtiles) {
@@ -320,22 +314,25 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
   // The transfer of tile t+3 is issued first, into the buffer tile t-1 has left. Past the
   // last tile the same instructions run on clamped tile indices and their results are
   // dropped, which keeps the loop body free of branches apart from the rare rescale.
-  dma_tile(0);
-  dma_tile(1);
-  dma_tile(2);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  __syncthreads();
-  load_kf(0);
+  // (RAGGED: none of it where the chunks are shorter than a tile of every quarter)
+  if (!RAGGED || ntiles > 0) {
+    dma_tile(0);
+    dma_tile(1);
+    dma_tile(2);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    __syncthreads();
+    load_kf(0);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) score_one(0, i);
+    for (int i = 0; i < 4; ++i) score_one(0, i);
 #pragma unroll
-  for (int tt = 0; tt < 2; ++tt)
+    for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      pk[1][tt][i] = (__bf16)0.0f;  // the first "previous" P V adds nothing
-      vf[0][tt][i] = (__bf16)0.0f;
-      vf[1][tt][i] = (__bf16)0.0f;
-    }
+      for (int i = 0; i < 8; ++i) {
+        pk[1][tt][i] = (__bf16)0.0f;  // the first "previous" P V adds nothing
+        vf[0][tt][i] = (__bf16)0.0f;
+        vf[1][tt][i] = (__bf16)0.0f;
+      }
+  }
 
 #define JG_FENCE() __builtin_amdgcn_sched_barrier(0)
   // One half of an iteration: query block `qa` has its scores ready and gets its softmax; the
@@ -345,14 +342,7 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
   // before the next half reads them (an MFMA chain of one wavefront shares the matrix core
   // with the other wavefront of the SIMD, so its last result arrives late); the two MFMAs in
   // front of the max are work for the matrix core while the vector unit runs the max tree.
-  // RAGGED: keys of the tile under the softmax from its first key to the chunk's end
-  int keys_left = p.sk - kq_u * qtiles * BN, soft_tile = 0;
   auto half = [&](int qa, int qo, auto&& after_scores, auto&& after_pv) {
-    if (RAGGED && keys_left < BN) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (8 * (i >> 2) + 4 * kg + (i & 3) >= keys_left) s[qa][i] = -INFINITY;
-    }
     score_one(qo, 0);
     score_one(qo, 1);
     JG_FENCE();
@@ -385,24 +375,78 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
     half(0, 1, [&]() { load_kf(nxt); }, [&]() { load_vf(cur); });
     // softmax of query block 1 (tile t) under: scores of block 0 (tile t+1), P V of block 0 (tile t)
     half(1, 0, [&]() {}, [&]() {});
-    if (RAGGED) {
-      keys_left -= BN;
-      if (++soft_tile == qtiles) {
-        soft_tile = 0;
-        keys_left += qtiles * BN;
-      }
-    }
     __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4): every transfer but this iteration's has landed
     __syncthreads();
   };
   // (unrolling over the four buffers would turn every LDS address into an immediate, but the
   // longer code ran no faster)
   for (int t = 0; t < ntiles; ++t) iteration(t & 3, (t + 1) & 3, (t + 3) & 3);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // the clamped transfers of the last iterations still target LDS
+  if (!RAGGED || ntiles > 0) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // the clamped transfers of the last iterations still target LDS
 #pragma unroll
-  for (int tt = 0; tt < 2; ++tt)
+    for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) pv_one(1, nb, tt);  // last tile, query block 1
+      for (int nb = 0; nb < 2; ++nb) pv_one(1, nb, tt);  // last tile, query block 1
+  }
+  // ---- the keys of every chunk behind its last multiple of 128: tile kq of them for quarter kq, two buffers
+  const int tail = RAGGED ? p.sk % (NQ * BN) : 0;
+  if (tail > 0) {
+    const int valid = tail - kq_u * BN;  // keys of this quarter's tile, <= 0: none
+    const int row = qtiles * NQ * BN + kq_u * BN + 16 * qg_u;
+    const uint32_t o0 = (uint32_t)min(row + (lane >> 3), p.sk - 1) * ROWB + dma_swz;
+    const uint32_t o1 = (uint32_t)min(row + 8 + (lane >> 3), p.sk - 1) * ROWB + dma_swz;
+    auto dma_tail = [&](int chunk, int buf) {
+      const uint32_t dst = lds_dma + (uint32_t)(buf * TILE_BYTES);
+      const char* kc = chunk_entry(0, chunk) + chunk_off;
+      const char* vc = chunk_entry(1, chunk) + chunk_off;
+      dma_1k(kc, o0, dst);
+      dma_1k(kc, o1, dst + 8 * ROWB);
+      dma_1k(vc, o0, dst + KV_BYTES);
+      dma_1k(vc, o1, dst + KV_BYTES + 8 * ROWB);
+    };
+    __syncthreads();  // every wavefront is past its last LDS read and its last transfer
+    dma_tail(0, 0);
+    for (int c = 0; c < p.nchunks; ++c) {
+      const int buf = c & 1;
+      asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // chunk c is here
+      // a V row past the end holds the last key's again, which must not meet a probability of 0 (it may be infinite):
+      // the lane that brought a piece of it clears the piece
+      unsigned char* mine = lds + buf * TILE_BYTES + KV_BYTES + 16 * qg * ROWB + lane * 16;
+      if (16 * qg + (lane >> 3) >= valid) *reinterpret_cast<u32x4*>(mine) = u32x4{0u, 0u, 0u, 0u};
+      if (16 * qg + 8 + (lane >> 3) >= valid) *reinterpret_cast<u32x4*>(mine + 8 * ROWB) = u32x4{0u, 0u, 0u, 0u};
+      __syncthreads();  // and every wavefront is done with the other buffer
+      if (c + 1 < p.nchunks) dma_tail(c + 1, buf ^ 1);
+      if (valid <= 0) continue;  // wave-uniform, the barriers are above
+      load_kf(buf);
+      load_vf(buf);
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) score_one(qb, i);
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (8 * (i >> 2) + 4 * kg + (i & 3) >= valid) s[qb][i] = -INFINITY;
+        new_max(qb);
+        const float mc = m[qb] * c2;
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+          float pr[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            pr[i] = __builtin_amdgcn_exp2f(s[qb][8 * tt + i] * c2 - mc);
+            l[qb][i & 1] += pr[i];
+          }
+          bf16x8 part[3];
+          parts8<true>(pr, part);
+#pragma unroll
+          for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+            for (int t = 2; t >= 0; --t)
+              o[qb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[nb][tt], part[t], o[qb][nb], 0, 0, 0);
+        }
+      }
+    }
+  }
 
   // ---- the two lanes of a query add their partial sums; the four key quarters combine via LDS
   // (quarters 1 and 3 hand over to 0 and 2, then 2 to 0)

@@ -42,6 +42,7 @@ using jg::BlockOf;
 using jg::ChunkTable;
 using jg::block_of;
 using jg::chunk_entry;
+using jg::parts8;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -212,6 +213,31 @@ __device__ __forceinline__ u32x2 pack4(float a, float b, float c, float d) {
   return r;
 }
 
+// c + a x v for eight fp32 values in B-fragment position, none of them rounded (see parts8). A bf16 fragment goes in
+// as it is; an fp16 one as two bf16 parts, which hold its 11 bits and its whole range.
+template <bool F16>
+__device__ __forceinline__ f32x16 mma_exact(typename Half<F16>::x8 a, const bf16x8 (&part)[3], f32x16 c) {
+  if constexpr (!F16) {
+#pragma unroll
+    for (int t = 2; t >= 0; --t) c = Half<false>::mma(a, part[t], c);
+  } else {
+    bf16x8 hi, lo;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float f = (float)a[e];
+      hi[e] = (__bf16)f;
+      const float h = (float)hi[e];
+      lo[e] = (__bf16)(f == h ? 0.0f : f - h);
+    }
+#pragma unroll
+    for (int t = 2; t >= 0; --t) {
+      c = Half<false>::mma(lo, part[t], c);
+      c = Half<false>::mma(hi, part[t], c);
+    }
+  }
+  return c;
+}
+
 // 16-byte piece `col` / 8 of a row in memory, zero past the head's columns
 template <int D, bool F16>
 __device__ __forceinline__ typename Half<F16>::x8 row_frag(const uint16_t* row, int col, int d) {
@@ -220,14 +246,14 @@ __device__ __forceinline__ typename Half<F16>::x8 row_frag(const uint16_t* row, 
   return __builtin_bit_cast(typename Half<F16>::x8, v);
 }
 
-// Which tile of which chunk a group takes next: tiles ks, ks + KS, ... of every chunk in turn. Every group makes
-// `steps` steps a chunk; in a step past the chunk's end rows_left is <= 0.
+// Which tile of which chunk a group takes next: tiles ks, ks + KS, ... of the rows lo .. hi - 1 of every chunk in turn.
+// Every group makes `steps` steps a chunk; in a step past the rows' end rows_left is <= 0.
 template <int KS>
 struct Stream {
-  int steps, rows, tile, step, chunk;
-  __device__ Stream(int rows_, int ks) : steps((rows_ + BT * KS - 1) / (BT * KS)), rows(rows_), tile(ks), step(0), chunk(0) {}
-  __device__ __forceinline__ int first_row() const { return tile * BT; }
-  __device__ __forceinline__ int rows_left() const { return rows - tile * BT; }
+  int steps, lo, hi, tile, step, chunk;
+  __device__ Stream(int lo_, int hi_, int ks) : steps((hi_ - lo_ + BT * KS - 1) / (BT * KS)), lo(lo_), hi(hi_), tile(ks), step(0), chunk(0) {}
+  __device__ __forceinline__ int first_row() const { return lo + tile * BT; }
+  __device__ __forceinline__ int rows_left() const { return hi - first_row(); }
   __device__ __forceinline__ void next() {
     tile += KS;
     if (++step == steps) {
@@ -252,11 +278,18 @@ struct Args {
   int sq, sk;            // sk: keys per chunk
   int d;                 // columns of a head, <= D and a multiple of 8
   int nchunks;
+  int exact_from;        // forward: first key of a chunk whose probabilities are not rounded (see exact_from())
   float scale;
 };
 
 // ------------------------------------------------------------------- forward
-template <int D, bool F16, int KS>
+// EXACT: some keys' probabilities are not rounded (p.exact_from < p.sk). A second loop and kernels of their own: with the
+// choice inside the one loop every tile took 4 to 10 % longer, with both loops in every kernel up to 7 % (head sizes 96
+// and 128, lengths that are multiples of 128).
+// What it costs, forward / backward of 64 heads x 100 queries x 8 chunks of 100 keys, rounded -> not: bf16, head size 64
+// 33 / 52 -> 34 / 58 us, 96 34 / 62 -> 40 / 78, 128 (127 keys) 35 / 86 -> 49 / 102; fp16, whose operands go in as two parts, 64
+// 34 / 52 -> 45 / 79. The one-thread-per-row kernels, which these chunks ran before, took 1107 / 2418 us at bf16 64, eight launches each way.
+template <int D, bool F16, int KS, bool EXACT>
 __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, Args p) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
@@ -283,78 +316,91 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
   for (int nb = 0; nb < G::NB; ++nb) o[nb] = zero16();
   float m = NO_SCORE, l = 0.0f;
 
-  TileRegs<D> rk;
-  TransRegs<D> rv;
-  Stream<KS> load(p.sk, ks), soft(p.sk, ks);
-  const int ntiles = load.steps * p.nchunks;
-  auto fetch = [&]() {
-    const uint16_t* kb = reinterpret_cast<const uint16_t*>(chunk_entry(0, load.chunk)) + chunk_off;
-    const uint16_t* vb = reinterpret_cast<const uint16_t*>(chunk_entry(1, load.chunk)) + chunk_off;
-    const long long at = (long long)load.first_row() * p.d;
-    tile_fetch<D>(rk, kb + at, tid, load.rows_left(), p.d);
-    trans_fetch<D>(rv, vb + at, tid, load.rows_left(), p.d);
-    load.next();
-  };
-  auto store = [&](int buf) {
-    tile_store_rows<D>(rk, lds + buf * BUF, tid);
-    trans_store<D>(rv, lds + buf * BUF + G::ROWMAJ, tid);
-  };
-  fetch();
-  store(0);
-  // The fragments that came straight from memory are waited for here, once. Left to the first matrix
-  // instruction that reads them, the wait sits inside the loop, behind the tile loads every iteration has
-  // just issued, and counts those too: each iteration then waited for its own prefetch.
 #pragma unroll
-  for (int c = 0; c < G::C16; ++c) asm volatile("" : "+v"(qf[c]));
-  __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
-    const unsigned char* kt = lds + (t & 1) * BUF;
-    const unsigned char* vt = kt + G::ROWMAJ;
-    if (t + 1 < ntiles) fetch();
-    // S^T: lane = query ln, register i = key 8*(i/4) + 4*kg + i%4 of the tile
-    f32x16 s = zero16();
+  for (int pass = 0; pass < (EXACT ? 2 : 1); ++pass) {
+    // the keys lo .. hi - 1 of every chunk
+    const bool exact = EXACT && pass == 1;
+    const int lo = exact ? p.exact_from : 0, hi = EXACT && !exact ? p.exact_from : p.sk;
+    if (EXACT && lo == hi) continue;
+    TileRegs<D> rk;
+    TransRegs<D> rv;
+    Stream<KS> load(lo, hi, ks), soft(lo, hi, ks);
+    const int ntiles = load.steps * p.nchunks;
+    auto fetch = [&]() {
+      const uint16_t* kb = reinterpret_cast<const uint16_t*>(chunk_entry(0, load.chunk)) + chunk_off;
+      const uint16_t* vb = reinterpret_cast<const uint16_t*>(chunk_entry(1, load.chunk)) + chunk_off;
+      const long long at = (long long)load.first_row() * p.d;
+      tile_fetch<D>(rk, kb + at, tid, load.rows_left(), p.d);
+      trans_fetch<D>(rv, vb + at, tid, load.rows_left(), p.d);
+      load.next();
+    };
+    auto store = [&](int buf) {
+      tile_store_rows<D>(rk, lds + buf * BUF, tid);
+      trans_store<D>(rv, lds + buf * BUF + G::ROWMAJ, tid);
+    };
+    fetch();
+    store(0);
+    // The fragments that came straight from memory are waited for here, once. Left to the first matrix
+    // instruction that reads them, the wait sits inside the loop, behind the tile loads every iteration has
+    // just issued, and counts those too: each iteration then waited for its own prefetch.
 #pragma unroll
-    for (int c = 0; c < G::C16; ++c)
-      s = Half<F16>::mma(frag<F16>(kt + ln * G::RP + (16 * c + 8 * kg) * 2), qf[c], s);
-    if (soft.rows_left() < BT) {  // wave-uniform
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (8 * (i >> 2) + 4 * kg + (i & 3) >= soft.rows_left()) s[i] = -INFINITY;
-    }
-    soft.next();
-    float mx = s[0];
-#pragma unroll
-    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mn = fmaxf(m, mx);
-    // the maximum settles after a few tiles: rescale only when some query of the wavefront saw a larger score
-    if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {
-      const float alpha = __builtin_amdgcn_exp2f((m - mn) * c2);  // first tile: 0
-      l *= alpha;
-#pragma unroll
-      for (int nb = 0; nb < G::NB; ++nb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[nb][i] *= alpha;
-      m = mn;
-    }
-    const float off = m * c2;
-    float pr[16], sum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      pr[i] = __builtin_amdgcn_exp2f(s[i] * c2 - off);
-      sum += pr[i];
-    }
-    l += sum;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const X8 pf = pack8<F16>(pr + 8 * ks);
-#pragma unroll
-      for (int nb = 0; nb < G::NB; ++nb)
-        o[nb] = Half<F16>::mma(frag<F16>(vt + (nb * 32 + ln) * G::TP + (16 * ks + 8 * kg) * 2), pf,
-                                                        o[nb]);
-    }
-    if (t + 1 < ntiles) store((t + 1) & 1);
+    for (int c = 0; c < G::C16; ++c) asm volatile("" : "+v"(qf[c]));
     __syncthreads();
+    for (int t = 0; t < ntiles; ++t) {
+      const unsigned char* kt = lds + (t & 1) * BUF;
+      const unsigned char* vt = kt + G::ROWMAJ;
+      if (t + 1 < ntiles) fetch();
+      // S^T: lane = query ln, register i = key 8*(i/4) + 4*kg + i%4 of the tile
+      f32x16 s = zero16();
+#pragma unroll
+      for (int c = 0; c < G::C16; ++c)
+        s = Half<F16>::mma(frag<F16>(kt + ln * G::RP + (16 * c + 8 * kg) * 2), qf[c], s);
+      if (soft.rows_left() < BT) {  // wave-uniform
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (8 * (i >> 2) + 4 * kg + (i & 3) >= soft.rows_left()) s[i] = -INFINITY;
+      }
+      soft.next();
+      float mx = s[0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float mn = fmaxf(m, mx);
+      // the maximum settles after a few tiles: rescale only when some query of the wavefront saw a larger score
+      if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {
+        const float alpha = __builtin_amdgcn_exp2f((m - mn) * c2);  // first tile: 0
+        l *= alpha;
+#pragma unroll
+        for (int nb = 0; nb < G::NB; ++nb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[nb][i] *= alpha;
+        m = mn;
+      }
+      const float off = m * c2;
+      float pr[16], sum = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        pr[i] = __builtin_amdgcn_exp2f(s[i] * c2 - off);
+        sum += pr[i];
+      }
+      l += sum;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const unsigned char* at = vt + ln * G::TP + (16 * ks + 8 * kg) * 2;
+        if (exact) {
+          bf16x8 part[3];
+          parts8<true>(pr + 8 * ks, part);
+#pragma unroll
+          for (int nb = 0; nb < G::NB; ++nb) o[nb] = mma_exact<F16>(frag<F16>(at + nb * 32 * G::TP), part, o[nb]);
+        } else {
+          const X8 pf = pack8<F16>(pr + 8 * ks);
+#pragma unroll
+          for (int nb = 0; nb < G::NB; ++nb) o[nb] = Half<F16>::mma(frag<F16>(at + nb * 32 * G::TP), pf, o[nb]);
+        }
+      }
+      if (t + 1 < ntiles) store((t + 1) & 1);
+      __syncthreads();
+    }
   }
   // the two lanes of a query saw the same maxima; their sums cover disjoint keys
   l += __shfl_xor(l, 32, 64);
@@ -428,7 +474,8 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
 }
 
 // ------------------------------------------------------------------- dQ (and delta)
-template <int D, bool F16, int KS>
+// EXACT (here and in the dK/dV kernel): dS and the probabilities are not rounded (chunks of fewer than EXACT_KEYS keys).
+template <int D, bool F16, int KS, bool EXACT>
 __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Args p) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
@@ -467,7 +514,7 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
 
   TileRegs<D> rk, rv;
   TransRegs<D> rkt;
-  Stream<KS> load(p.sk, ks), soft(p.sk, ks);
+  Stream<KS> load(0, p.sk, ks), soft(0, p.sk, ks);
   const int ntiles = load.steps * p.nchunks;
   auto fetch = [&]() {
     const long long at = chunk_off + (long long)load.first_row() * p.d;
@@ -512,11 +559,17 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
     for (int i = 0; i < 16; ++i) ds[i] = __builtin_amdgcn_exp2f(s[i] * c2 - lse2) * (dp[i] - delta);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      const X8 dsf = pack8<F16>(ds + 8 * ks);
+      const unsigned char* at = ktt + ln * G::TP + (16 * ks + 8 * kg) * 2;
+      if constexpr (EXACT) {
+        bf16x8 part[3];
+        parts8<false>(ds + 8 * ks, part);
 #pragma unroll
-      for (int nb = 0; nb < G::NB; ++nb)
-        dq[nb] = Half<F16>::mma(frag<F16>(ktt + (nb * 32 + ln) * G::TP + (16 * ks + 8 * kg) * 2),
-                                                         dsf, dq[nb]);
+        for (int nb = 0; nb < G::NB; ++nb) dq[nb] = mma_exact<F16>(frag<F16>(at + nb * 32 * G::TP), part, dq[nb]);
+      } else {
+        const X8 dsf = pack8<F16>(ds + 8 * ks);
+#pragma unroll
+        for (int nb = 0; nb < G::NB; ++nb) dq[nb] = Half<F16>::mma(frag<F16>(at + nb * 32 * G::TP), dsf, dq[nb]);
+      }
     }
     if (t + 1 < ntiles) store((t + 1) & 1);
     __syncthreads();
@@ -556,7 +609,7 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
 // that way), so head sizes above 96 run the kernel twice: MODE 1 forms dV only (from P), MODE 2 dK only
 // (from dS), each with one accumulator and two workgroups per CU; the scores are computed in both.
 // A launch with no more workgroups than CUs gains nothing from that and keeps the single pass.
-template <int D, bool F16, int MODE, int KS>
+template <int D, bool F16, int MODE, int KS, bool EXACT>
 __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 : 1) void attn_wide_dkv_kernel(ChunkTable, Args p) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
@@ -599,7 +652,7 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
   TransRegs<D> rqt, rgt;     // Q^T (dK only); dO^T (dV only)
   float st = 0.0f;  // one statistic per thread of the group's first wavefront: lse2 (lanes 0-31) or delta (32-63)
   int st_rows = 0;  // rows of the tile it belongs to
-  Stream<KS> load(p.sq, ks);
+  Stream<KS> load(0, p.sq, ks);
   const int ntiles = load.steps;
   auto fetch = [&]() {
     const long long at = (long long)load.first_row() * p.d;
@@ -665,17 +718,30 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
     }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      if (DV) {
-        const X8 pf = pack8<F16>(pr + 8 * ks);
+      const int at = ln * G::TP + (16 * ks + 8 * kg) * 2;
+      if constexpr (EXACT) {
+        bf16x8 part[3];
+        if (DV) {
+          parts8<true>(pr + 8 * ks, part);
 #pragma unroll
-        for (int nb = 0; nb < G::NB; ++nb)
-          dv[nb] = Half<F16>::mma(frag<F16>(gtt + (nb * 32 + ln) * G::TP + (16 * ks + 8 * kg) * 2), pf, dv[nb]);
-      }
-      if (DK) {
-        const X8 dsf = pack8<F16>(ds + 8 * ks);
+          for (int nb = 0; nb < G::NB; ++nb) dv[nb] = mma_exact<F16>(frag<F16>(gtt + at + nb * 32 * G::TP), part, dv[nb]);
+        }
+        if (DK) {
+          parts8<false>(ds + 8 * ks, part);
 #pragma unroll
-        for (int nb = 0; nb < G::NB; ++nb)
-          dk[nb] = Half<F16>::mma(frag<F16>(qtt + (nb * 32 + ln) * G::TP + (16 * ks + 8 * kg) * 2), dsf, dk[nb]);
+          for (int nb = 0; nb < G::NB; ++nb) dk[nb] = mma_exact<F16>(frag<F16>(qtt + at + nb * 32 * G::TP), part, dk[nb]);
+        }
+      } else {
+        if (DV) {
+          const X8 pf = pack8<F16>(pr + 8 * ks);
+#pragma unroll
+          for (int nb = 0; nb < G::NB; ++nb) dv[nb] = Half<F16>::mma(frag<F16>(gtt + at + nb * 32 * G::TP), pf, dv[nb]);
+        }
+        if (DK) {
+          const X8 dsf = pack8<F16>(ds + 8 * ks);
+#pragma unroll
+          for (int nb = 0; nb < G::NB; ++nb) dk[nb] = Half<F16>::mma(frag<F16>(qtt + at + nb * 32 * G::TP), dsf, dk[nb]);
+        }
       }
     }
     if (t + 1 < ntiles) store((t + 1) & 1);
@@ -753,7 +819,7 @@ int launch(K kernel, dim3 grid, int threads, int lds, const ChunkTable& tab, con
   return JG_OK;
 }
 
-template <int D, bool F16>
+template <int D, bool F16, bool EXACT>
 int launch_fwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
   typedef Geo<D> G;
   constexpr int LDS = 2 * (G::ROWMAJ + G::TRANS);
@@ -761,12 +827,12 @@ int launch_fwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_
   const char* who = "jg_attn_fwd(wide)";
   const int ks = split_of((long long)grid.x * batch, D <= 64 ? 4 : 2);
   if constexpr (D <= 64)
-    if (ks == 4) return launch(&attn_wide_fwd_kernel<D, F16, 4>, grid, 4 * GROUP, 4 * LDS, tab, a, s, who);
-  if (ks == 2) return launch(&attn_wide_fwd_kernel<D, F16, 2>, grid, 2 * GROUP, 2 * LDS, tab, a, s, who);
-  return launch(&attn_wide_fwd_kernel<D, F16, 1>, grid, GROUP, LDS, tab, a, s, who);
+    if (ks == 4) return launch(&attn_wide_fwd_kernel<D, F16, 4, EXACT>, grid, 4 * GROUP, 4 * LDS, tab, a, s, who);
+  if (ks == 2) return launch(&attn_wide_fwd_kernel<D, F16, 2, EXACT>, grid, 2 * GROUP, 2 * LDS, tab, a, s, who);
+  return launch(&attn_wide_fwd_kernel<D, F16, 1, EXACT>, grid, GROUP, LDS, tab, a, s, who);
 }
 
-template <int D, bool F16>
+template <int D, bool F16, bool EXACT>
 int launch_bwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
   typedef Geo<D> G;
   constexpr int DQ_LDS = 2 * (2 * G::ROWMAJ + G::TRANS);
@@ -776,21 +842,22 @@ int launch_bwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_
   const long long dkv_workgroups = (long long)dkv_grid.x * batch * a.nchunks;
   const char* who = "jg_attn_bwd(wide, dq)";
   int rc = split_of((long long)dq_grid.x * batch, 2) == 2
-               ? launch(&attn_wide_dq_kernel<D, F16, 2>, dq_grid, 2 * GROUP, 2 * DQ_LDS, tab, a, s, who)
-               : launch(&attn_wide_dq_kernel<D, F16, 1>, dq_grid, GROUP, DQ_LDS, tab, a, s, who);
+               ? launch(&attn_wide_dq_kernel<D, F16, 2, EXACT>, dq_grid, 2 * GROUP, 2 * DQ_LDS, tab, a, s, who)
+               : launch(&attn_wide_dq_kernel<D, F16, 1, EXACT>, dq_grid, GROUP, DQ_LDS, tab, a, s, who);
   if (rc != JG_OK) return rc;
   who = "jg_attn_bwd(wide, dkv)";
-  // up to head size 96: dK and dV in one pass; above: one pass each when the launch has more workgroups than the
-  // chip has CUs (register budget, see the kernel)
-  if constexpr (D <= 96) {
+  // up to head size 96 (64 with EXACT): dK and dV in one pass; above: one pass each when the launch has more workgroups
+  // than the chip has CUs, and with EXACT always (register budget, see the kernel)
+  if constexpr (D <= (EXACT ? 64 : 96)) {
     if (split_of(dkv_workgroups, 2) == 2)
-      return launch(&attn_wide_dkv_kernel<D, F16, 0, 2>, dkv_grid, 2 * GROUP, 2 * DKV_LDS, tab, a, s, who);
-  } else if (dkv_workgroups > cu_count()) {
-    rc = launch(&attn_wide_dkv_kernel<D, F16, 1, 1>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
+      return launch(&attn_wide_dkv_kernel<D, F16, 0, 2, EXACT>, dkv_grid, 2 * GROUP, 2 * DKV_LDS, tab, a, s, who);
+  } else if (EXACT || dkv_workgroups > cu_count()) {
+    rc = launch(&attn_wide_dkv_kernel<D, F16, 1, 1, EXACT>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
     if (rc != JG_OK) return rc;
-    return launch(&attn_wide_dkv_kernel<D, F16, 2, 1>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
+    return launch(&attn_wide_dkv_kernel<D, F16, 2, 1, EXACT>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
   }
-  return launch(&attn_wide_dkv_kernel<D, F16, 0, 1>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
+  if constexpr (D <= 64 || !EXACT) return launch(&attn_wide_dkv_kernel<D, F16, 0, 1, EXACT>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
+  return JG_OK;
 }
 
 // f(D constant, F16 constant) for the narrowest kernel that holds the head
@@ -822,8 +889,11 @@ int attn_wide_fwd_chunks(void* out, float* lse, const void* q, const void* const
   a.out_acc = out_acc;
   a.lse_acc = lse_acc;
   a.sq = sq; a.sk = sk; a.d = d; a.nchunks = nchunks; a.scale = scale;
+  a.exact_from = exact_from(sk, d, dtype);
   const ChunkTable tab = chunk_table(k, v, nullptr, nullptr, nchunks);
-  return by_width(d, dtype, [&](auto width, auto f16) { return launch_fwd<width(), f16()>(tab, a, batch, s); });
+  return by_width(d, dtype, [&](auto width, auto f16) {
+    return a.exact_from < sk ? launch_fwd<width(), f16(), true>(tab, a, batch, s) : launch_fwd<width(), f16(), false>(tab, a, batch, s);
+  });
 }
 
 int attn_wide_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q, const void* const* k,
@@ -838,7 +908,9 @@ int attn_wide_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
   a.dq = static_cast<uint16_t*>(dq);
   a.sq = sq; a.sk = sk; a.d = d; a.nchunks = nchunks; a.scale = scale;
   const ChunkTable tab = chunk_table(k, v, dk, dv, nchunks);
-  return by_width(d, dtype, [&](auto width, auto f16) { return launch_bwd<width(), f16()>(tab, a, batch, s); });
+  return by_width(d, dtype, [&](auto width, auto f16) {
+    return sk < EXACT_KEYS ? launch_bwd<width(), f16(), true>(tab, a, batch, s) : launch_bwd<width(), f16(), false>(tab, a, batch, s);
+  });
 }
 
 }  // namespace jg

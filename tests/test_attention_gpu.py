@@ -516,3 +516,87 @@ def test_ring_of_any_lengths_in_one_pass(b, h, sq, sk, d, P, dtype, dev):
     o_j, l_j = ja.core_forward(q, ks[0], vs[0], scale)
     acc2, l2 = ja.fused_online_softmax_merge_(acc2, l2, o_j, l_j, "bhsd")
     assert rel_l2(acc1, acc2) < 1e-5 and rel_l2(l1, l2) < 1e-5
+
+
+def _differ(a, b) -> float:
+    return (a != b).double().mean().item()
+
+
+# Two fp32 evaluations differ by about 4e-6 of a value, and 16-bit values lie 2^-8 (bf16) and 2^-11 (fp16) of it apart, so up
+# to 0.2 % and 1.6 % of the rounded results may differ; with probabilities rounded to 16 bits more than a third do.
+_STRAYS = {torch.bfloat16: 0.005, torch.float16: 0.02}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("h,sq,sk,d,P", [(4, 100, 100, 64, 2), (4, 300, 127, 64, 3), (3, 64, 31, 64, 1), (4, 100, 65, 40, 2), (3, 130, 97, 32, 5),
+                                         (3, 130, 97, 96, 2), (3, 200, 127, 128, 2), (300, 130, 100, 80, 1)], ids=str)
+def test_short_key_ranges_keep_probabilities_in_fp32(h, sq, sk, d, P, dtype, dev):
+    """Fewer than 128 keys a chunk: the same results as the one-thread-per-row kernels (a bias of zeros selects them), which
+    hold probabilities and dS in fp32, forward and backward, and over the chunks of a ring."""
+    torch.manual_seed(sk + d)
+    mk = lambda n: torch.randn(1, h, n, d, device=dev).to(dtype)  # noqa: E731
+    q, dout, ks, vs, scale = mk(sq), mk(sq), [mk(sk) for _ in range(P)], [mk(sk) for _ in range(P)], d**-0.5
+    out, lse = ja.ring_forward(q, ks, vs, scale)
+    k, v = torch.cat(ks, -2), torch.cat(vs, -2)
+    zeros = torch.zeros(sq, sk * P, device=dev)
+    want_o, want_l = ja.core_forward(q, k, v, scale, bias=zeros)
+    assert _differ(out, want_o) < _STRAYS[dtype] and rel_l2(lse, want_l) < 1e-6
+    dq, dks, dvs = ja.ring_backward(dout, q, want_o, want_l, ks, vs, scale)
+    want = ja.core_backward(dout, q, k, v, want_o, want_l, scale, bias=zeros)
+    for got, w in zip((dq, torch.cat(dks, -2), torch.cat(dvs, -2)), want):
+        assert _differ(got, w) < _STRAYS[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("h,sq,sk,d,P", [(3, 130, 300, 64, 1), (3, 256, 1000, 64, 3), (30, 256, 1000, 128, 2), (3, 130, 255, 96, 3)], ids=str)
+def test_keys_behind_the_last_whole_tile_keep_probabilities_in_fp32(h, sq, sk, d, P, dtype, dev):
+    """Forward at a head size that fills a kernel: the keys of a chunk behind its last multiple of 128. The whole tiles
+    have probabilities near 0 here, so that the last keys alone make the result."""
+    if dtype == torch.float16 and d == 64:
+        pytest.skip("fp16 heads of 64 columns fill no kernel of their own")
+    torch.manual_seed(sk + d)
+    mk = lambda n: torch.randn(1, h, n, d, device=dev).to(dtype)  # noqa: E731
+    q, k, vs, scale = mk(sq), mk(sk), [mk(sk) for _ in range(P)], d**-0.5
+    q[..., 0], k[..., 0] = 16, 0
+    k[:, :, : sk // 128 * 128, 0] = -8 * d**0.5  # scores of -128 and below
+    out, lse = ja.ring_forward(q, [k] * P, vs, scale)
+    want_o, want_l = ja.core_forward(q, torch.cat([k] * P, -2), torch.cat(vs, -2), scale, bias=torch.zeros(sq, sk * P, device=dev))
+    assert _differ(out, want_o) < _STRAYS[dtype] and rel_l2(lse, want_l) < 1e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("sq,sk,d", [(70, 100, 64), (70, 1000, 64), (70, 100, 128), (70, 200, 96), (70, 33, 32)], ids=str)
+def test_infinite_values_stay_infinite_where_probabilities_are_kept_in_fp32(sq, sk, d, dtype, dev):
+    """A value that is infinite makes its output column infinite, not NaN, also as the last key of a range."""
+    torch.manual_seed(sk)
+    q, k, v = (torch.randn(1, 2, n, d, device=dev).to(dtype) for n in (sq, sk, sk))
+    v[..., sk - 1, 3], v[..., sk // 2, 5] = float("inf"), float("-inf")
+    out, _ = ja.core_forward(q, k, v, d**-0.5)
+    want, _ = ja.core_forward(q, k, v, d**-0.5, bias=torch.zeros(sq, sk, device=dev))
+    assert torch.isinf(want[..., 3]).all() and torch.isinf(want[..., 5]).all()
+    assert torch.equal(out[..., (3, 5)], want[..., (3, 5)]) and torch.isfinite(out[..., 6:]).all()
+
+
+@pytest.mark.parametrize("sk", [100, 200, 256])
+def test_misaligned_heads_of_64_run_the_kernels_that_take_any_alignment(sk, dev):
+    """The C entry points on tensors that start 2 bytes off a 16-byte boundary: the one-thread-per-row kernels."""
+    from jigsaw_amd import _lib
+
+    torch.manual_seed(sk)
+    lib, h, sq, d, scale = _lib.load(), 2, 130, 64, 0.125
+    off = lambda *s: torch.randn(h * s[0] * s[1] + 1, device=dev).bfloat16()[1:].view(h, *s)  # noqa: E731
+    q, dout, k, v, out, dq, dk, dv = off(sq, d), off(sq, d), off(sk, d), off(sk, d), off(sq, d), off(sq, d), off(sk, d), off(sk, d)
+    lse = torch.empty(h, sq, device=dev)
+    ws = torch.empty(int(lib.jg_attn_bwd_workspace_bytes(h, sq, sk, d)), dtype=torch.uint8, device=dev)
+    p, bf16, stream = _lib.ptr, _lib.dtype_code(torch.bfloat16), _lib.stream_ptr(q.device)
+    _lib.check(lib.jg_attn_fwd(p(out), p(lse), p(q), p(k), p(v), h, sq, sk, d, scale, None, 0, None, None, bf16, stream))
+    _lib.check(lib.jg_attn_bwd(p(dq), p(dk), p(dv), p(dout), p(q), p(k), p(v), p(out), p(lse), h, sq, sk, d, scale, None, 0, None, bf16,
+                               p(ws), ws.numel(), stream))
+    want_o, want_l = ja.core_forward(q.clone(), k.clone(), v.clone(), scale, bias=torch.zeros(sq, sk, device=dev))
+    want = ja.core_backward(dout, q, k, v, want_o, want_l, scale, bias=torch.zeros(sq, sk, device=dev))
+    assert torch.equal(out, want_o) and torch.equal(lse, want_l)
+    for got, w in zip((dq, dk, dv), want):
+        assert torch.equal(got, w)
+    acc = torch.zeros(h, sq, d, device=dev)
+    rc = lib.jg_attn_fwd(None, None, p(q), p(k), p(v), h, sq, sk, d, scale, None, 0, p(acc), p(lse), bf16, stream)
+    assert rc == -2
