@@ -343,6 +343,11 @@ int jg_gn_moments(float* mean, float* sq, float* count_sum, const void* x, int64
 int jg_gn_apply(void* y, void* x_norm, const void* x, const float* mean, const float* rstd,
                 const void* weight, const void* bias, int64_t batch, int64_t channels,
                 int64_t spatial, int64_t groups, int dtype, void* stream);
+/* The same without x_norm, and x_kept = a copy of x (NULL: none), made on the way: what a backward from x needs where
+ * the caller may change x in between. */
+int jg_gn_apply_keep(void* y, void* x_kept, const void* x, const float* mean, const float* rstd,
+                     const void* weight, const void* bias, int64_t batch, int64_t channels,
+                     int64_t spatial, int64_t groups, int dtype, void* stream);
 
 /* Backward partials (_functional.py:438-462), one pass over g and x_norm:
  *   gsum[n][grp]  = sum of g * weight[c]            over the group, local positions
@@ -369,6 +374,10 @@ int jg_gn_bwd_apply_x(void* gx, const void* g, const void* x, const void* weight
 int jg_gn_forward(void* y, float* mean, float* rstd, const void* x, const void* weight, const void* bias, int64_t batch,
                   int64_t channels, int64_t spatial, int64_t groups, float eps, int dtype, void* workspace,
                   size_t workspace_bytes, void* stream);
+/* jg_gn_forward with x_kept as in jg_gn_apply_keep. */
+int jg_gn_forward_keep(void* y, void* x_kept, float* mean, float* rstd, const void* x, const void* weight, const void* bias,
+                       int64_t batch, int64_t channels, int64_t spatial, int64_t groups, float eps, int dtype,
+                       void* workspace, size_t workspace_bytes, void* stream);
 int jg_gn_backward(void* gx, void* gw, void* gb, const void* g, const void* x, const float* mean, const float* rstd,
                    const void* weight, int64_t batch, int64_t channels, int64_t spatial, int64_t groups, int dtype,
                    int grad_dtype, void* workspace, size_t workspace_bytes, void* stream);

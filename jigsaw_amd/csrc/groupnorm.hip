@@ -9,11 +9,12 @@
 // sample of the block's own elements; normalise + affine), backward two (the sums; the input
 // gradient), both from x and the statistics, x_hat recomputed in fp32 on the way. x_hat itself
 // is only written for a caller that asks for it (jg_gn_apply with x_norm, jg_gn_partial_bwd,
-// jg_gn_bwd_apply): that is one more tensor written and two read, and it is rounded. On
-// 8 x 64 x 1024^2 bf16, 8 groups (1.07 GB a tensor) forward + backward is 1.54 ms = 5.6 TB/s over
-// eight tensors, what a copy reaches; 2.01 ms with three passes forward and x_hat stored. Both
-// passes of a sample before the next one, to find its tensor in the last-level cache, were
-// tried: 1.66 ms (eight launches that are each too small to fill the memory system).
+// jg_gn_bwd_apply): it is rounded, and the backward is less exact from it. A step whose backward takes x
+// keeps a copy of it (jg_gn_apply_keep, jg_gn_forward_keep), which the second pass writes beside y: the caller
+// may change x before the backward. On 8 x 64 x 1024^2 bf16, 8 groups (1.07 GB a tensor) forward +
+// backward is 1.80 ms = 5.4 TB/s over nine tensors, what a copy reaches; 1.55 ms without the copy, 2.17 ms with
+// three passes forward and x_hat stored. Both passes of a sample before the next one, to find its tensor in the
+// last-level cache, were tried: 0.12 ms more (eight launches that are each too small to fill the memory system).
 // Rows and spans start anywhere (S need not be a multiple of 8): a block takes the whole 16-byte
 // words of its range as vectors and the elements before the first and behind the last one by one.
 //
@@ -299,6 +300,7 @@ __global__ __launch_bounds__(64) void gn_bwd_finish_kernel(float* __restrict__ s
 struct ApplyArgs {
   void* out;         // y / gx
   void* out_norm;    // forward: x_norm, or NULL
+  void* out_kept;    // forward: x once more, or NULL
   const void* in;    // x / g
   const void* in2;   // backward: x_norm (FROM_X: x)
   const float* mean; // forward and FROM_X
@@ -334,6 +336,7 @@ __global__ __launch_bounds__(kThreads) void gn_apply_kernel(ApplyArgs p, long lo
   const T* in2 = static_cast<const T*>(p.in2);
   T* out = static_cast<T*>(p.out);
   T* norm = static_cast<T*>(p.out_norm);
+  T* kept = static_cast<T*>(p.out_kept);
   // forward: (y, x_norm): x_norm is rounded to the compute dtype and y computed from the rounded value, as the
   // reference computes y from the x_norm tensor
   auto forward = [&](float v, float& xn) {
@@ -350,6 +353,7 @@ __global__ __launch_bounds__(kThreads) void gn_apply_kernel(ApplyArgs p, long lo
     }
 #pragma unroll
     for (int q = 0; q < count(); ++q) {
+      if (!BWD && kept != nullptr) store_vec<DT>(kept + i + q * step, v[q]);
 #pragma unroll
       for (int t = 0; t < V; ++t) v[q][t] = BWD ? backward(v[q][t], x[q][t]) : forward(v[q][t], x[q][t]);
       if (!BWD && norm != nullptr) store_vec<DT>(norm + i + q * step, x[q]);
@@ -363,6 +367,7 @@ __global__ __launch_bounds__(kThreads) void gn_apply_kernel(ApplyArgs p, long lo
                  float xn = BWD ? Elem<DT>::up(in2[i]) : 0.0f;
                  const float r = BWD ? backward(v, xn) : forward(v, xn);
                  if (!BWD && norm != nullptr) norm[i] = Elem<DT>::down(xn);
+                 if (!BWD && kept != nullptr) kept[i] = in[i];
                  out[i] = Elem<DT>::down(r);
                });
 }
@@ -457,7 +462,7 @@ int apply_launch(const ApplyArgs& a, long long N, long long S, hipStream_t s, co
   const long long rows = N * a.C;
   if (rows == 0 || S == 0) return JG_OK;
   const int chunks = chunks_of(S);
-  const bool vec_ok = aligned16(a.out) && aligned16(a.in) && aligned16(a.in2) && aligned16(a.out_norm);
+  const bool vec_ok = aligned16(a.out) && aligned16(a.in) && aligned16(a.in2) && aligned16(a.out_norm) && aligned16(a.out_kept);
   gn_apply_kernel<DT, BWD, FROM_X><<<(unsigned)(rows * chunks), kThreads, 0, s>>>(a, S, chunks, chunk_len_of(S, chunks), vec_ok);
   JG_CHECK_LAUNCH(who);
   return JG_OK;
@@ -528,31 +533,42 @@ extern "C" int jg_gn_moments(float* mean, float* sq, float* count_sum, const voi
 #undef CALL
 }
 
-extern "C" int jg_gn_apply(void* y, void* x_norm, const void* x, const float* mean, const float* rstd,
-                           const void* weight, const void* bias, int64_t batch, int64_t channels,
-                           int64_t spatial, int64_t groups, int dtype, void* stream) {
-  const char* who = "jg_gn_apply";
+static int apply_forward(const char* who, void* y, void* x_norm, void* x_kept, const void* x, const float* mean, const float* rstd,
+                         const void* weight, const void* bias, int64_t batch, int64_t channels, int64_t spatial,
+                         int64_t groups, int dtype, void* stream) {
   int rc = check(who, batch, channels, spatial, groups, dtype);
   if (rc) return rc;
   JG_REQUIRE(y && x && mean && rstd, "%s: NULL pointer", who);
   hipStream_t s = static_cast<hipStream_t>(stream);
   ApplyArgs a = {};
-  a.out = y; a.out_norm = x_norm; a.in = x; a.mean = mean; a.rstd = rstd; a.weight = weight; a.bias = bias;
+  a.out = y; a.out_norm = x_norm; a.out_kept = x_kept; a.in = x; a.mean = mean; a.rstd = rstd; a.weight = weight; a.bias = bias;
   a.C = (int)channels; a.G = (int)groups;
 #define CALL(DT) apply_launch<DT, false, true>(a, batch, spatial, s, who)
   JG_GN_DISPATCH(CALL)
 #undef CALL
 }
 
+extern "C" int jg_gn_apply(void* y, void* x_norm, const void* x, const float* mean, const float* rstd,
+                           const void* weight, const void* bias, int64_t batch, int64_t channels,
+                           int64_t spatial, int64_t groups, int dtype, void* stream) {
+  return apply_forward("jg_gn_apply", y, x_norm, nullptr, x, mean, rstd, weight, bias, batch, channels, spatial, groups, dtype, stream);
+}
+
+extern "C" int jg_gn_apply_keep(void* y, void* x_kept, const void* x, const float* mean, const float* rstd,
+                                const void* weight, const void* bias, int64_t batch, int64_t channels,
+                                int64_t spatial, int64_t groups, int dtype, void* stream) {
+  return apply_forward("jg_gn_apply_keep", y, nullptr, x_kept, x, mean, rstd, weight, bias, batch, channels, spatial, groups, dtype, stream);
+}
+
 // Both passes of the forward / of the backward for a tensor that one rank holds whole.
 namespace {
 template <int DT>
-int forward_all(void* y, float* mean, float* rstd, const void* x, const void* weight, const void* bias, long long N,
+int forward_all(void* y, void* x_kept, float* mean, float* rstd, const void* x, const void* weight, const void* bias, long long N,
                 long long C, long long S, long long G, float eps, float* ws, hipStream_t s, const char* who) {
   int rc = moments_launch<DT>(mean, nullptr, nullptr, rstd, x, N * G, C / G * S, eps, ws, s, who);
   if (rc) return rc;
   ApplyArgs a = {};
-  a.out = y; a.in = x; a.mean = mean; a.rstd = rstd; a.weight = weight; a.bias = bias; a.C = (int)C; a.G = (int)G;
+  a.out = y; a.out_kept = x_kept; a.in = x; a.mean = mean; a.rstd = rstd; a.weight = weight; a.bias = bias; a.C = (int)C; a.G = (int)G;
   return apply_launch<DT, false, true>(a, N, S, s, who);
 }
 
@@ -574,13 +590,20 @@ int backward_all(void* gx, void* gw, void* gb, int wdtype, const void* g, const 
 extern "C" int jg_gn_forward(void* y, float* mean, float* rstd, const void* x, const void* weight, const void* bias,
                              int64_t batch, int64_t channels, int64_t spatial, int64_t groups, float eps, int dtype,
                              void* workspace, size_t workspace_bytes, void* stream) {
+  return jg_gn_forward_keep(y, nullptr, mean, rstd, x, weight, bias, batch, channels, spatial, groups, eps, dtype, workspace,
+                            workspace_bytes, stream);
+}
+
+extern "C" int jg_gn_forward_keep(void* y, void* x_kept, float* mean, float* rstd, const void* x, const void* weight,
+                                  const void* bias, int64_t batch, int64_t channels, int64_t spatial, int64_t groups,
+                                  float eps, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
   const char* who = "jg_gn_forward";
   int rc = check(who, batch, channels, spatial, groups, dtype);
   if (rc) return rc;
   JG_REQUIRE(y && mean && rstd && x, "%s: NULL pointer", who);
   if ((rc = check_ws(who, workspace, workspace_bytes, batch, channels, spatial))) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define CALL(DT) forward_all<DT>(y, mean, rstd, x, weight, bias, batch, channels, spatial, groups, eps, static_cast<float*>(workspace), s, who)
+#define CALL(DT) forward_all<DT>(y, x_kept, mean, rstd, x, weight, bias, batch, channels, spatial, groups, eps, static_cast<float*>(workspace), s, who)
   JG_GN_DISPATCH(CALL)
 #undef CALL
 }

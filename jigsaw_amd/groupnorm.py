@@ -176,13 +176,17 @@ class _GroupNorm(torch.autograd.Function):
 
 
 class _GroupNormOutput(torch.autograd.Function):
-    """``_GroupNorm`` for a caller that wants ``y`` alone: ``x`` and the statistics are kept for the backward instead of
-    ``x_norm``, which is then neither written nor read (the backward recomputes it, unrounded, on the way)."""
+    """``_GroupNorm`` for a caller that wants ``y`` alone: the backward takes ``x`` and the statistics instead of ``x_norm``,
+    which it recomputes, unrounded, on the way. It takes a copy of ``x`` of its own, which the pass that writes ``y`` makes
+    where a backward can follow: the caller may change ``x`` in place in between (``x += group_norm(x, ...)``), as
+    it may where ``x_norm`` is kept."""
 
     @staticmethod
-    def forward(ctx, x, num_groups, weight, bias, spatial_groups, eps):  # noqa: D102
+    def forward(ctx, x, num_groups, weight, bias, spatial_groups, eps, grad):  # noqa: D102
         cdt = _compute_dtype(x)
-        x = x.to(cdt).contiguous()
+        given, x = x, x.to(cdt).contiguous()
+        # a cast or a rearrangement is a copy already
+        kept = torch.empty_like(x) if grad and any(ctx.needs_input_grad) and x.data_ptr() == given.data_ptr() else None
         w = None if weight is None else weight.to(cdt).contiguous()
         b = None if bias is None else bias.to(cdt).contiguous()
         n, c, s = _dims(x)
@@ -190,19 +194,20 @@ class _GroupNormOutput(torch.autograd.Function):
         y = torch.empty_like(x)
         if spatial_groups:
             mean, rstd, count = _global_statistics(x, num_groups, spatial_groups, eps)
-            rc = lib.jg_gn_apply(_lib.ptr(y), None, _lib.ptr(x), _lib.ptr(mean), _lib.ptr(rstd), _lib.ptr(w), _lib.ptr(b),
-                                 n, c, s, num_groups, code, _lib.stream_ptr(dev))
-            _lib.check(rc, "jg_gn_apply")
+            rc = lib.jg_gn_apply_keep(_lib.ptr(y), _lib.ptr(kept), _lib.ptr(x), _lib.ptr(mean), _lib.ptr(rstd), _lib.ptr(w),
+                                      _lib.ptr(b), n, c, s, num_groups, code, _lib.stream_ptr(dev))
+            _lib.check(rc, "jg_gn_apply_keep")
         else:
             mean, rstd = torch.empty(2, n, num_groups, dtype=torch.float32, device=dev).unbind(0)
             count = None
             ws, nbytes = _workspace(lib, n, c, s, dev)
-            rc = lib.jg_gn_forward(_lib.ptr(y), _lib.ptr(mean), _lib.ptr(rstd), _lib.ptr(x), _lib.ptr(w), _lib.ptr(b), n, c, s,
-                                   num_groups, float(eps), code, _lib.ptr(ws), nbytes, _lib.stream_ptr(dev))
-            _lib.check(rc, "jg_gn_forward")
+            rc = lib.jg_gn_forward_keep(_lib.ptr(y), _lib.ptr(kept), _lib.ptr(mean), _lib.ptr(rstd), _lib.ptr(x), _lib.ptr(w),
+                                        _lib.ptr(b), n, c, s, num_groups, float(eps), code, _lib.ptr(ws), nbytes,
+                                        _lib.stream_ptr(dev))
+            _lib.check(rc, "jg_gn_forward_keep")
         ctx.num_groups, ctx.spatial_groups = num_groups, spatial_groups
         ctx.dtypes = (None if weight is None else weight.dtype, None if bias is None else bias.dtype)
-        ctx.save_for_backward(x, mean, rstd, count, w)
+        ctx.save_for_backward(x if kept is None else kept, mean, rstd, count, w)
         return y
 
     @staticmethod
@@ -240,7 +245,7 @@ class _GroupNormOutput(torch.autograd.Function):
                 rc = lib.jg_gn_bwd_apply_x(_lib.ptr(gx), _lib.ptr(g), _lib.ptr(x), _lib.ptr(w), _lib.ptr(mean), _lib.ptr(rstd),
                                            _lib.ptr(sums), _lib.ptr(count), n, c, s, groups, code, stream)
                 _lib.check(rc, "jg_gn_bwd_apply_x")
-        return gx, None, None if gw is None else gw.to(dt_w), None if gb is None else gb.to(dt_b), None, None
+        return gx, None, None if gw is None else gw.to(dt_w), None if gb is None else gb.to(dt_b), None, None, None
 
 
 def group_norm(x, num_groups, weight=None, bias=None, spatial_groups=(), eps=1e-5):
@@ -252,7 +257,7 @@ def group_norm(x, num_groups, weight=None, bias=None, spatial_groups=(), eps=1e-
     if x.numel() == 0:
         return _GroupNorm.apply(x, num_groups, weight, bias, spatial_groups, eps)[0]
     split = tuple(g for g in spatial_groups or () if g is not None and int(g.size()) > 1)
-    return _GroupNormOutput.apply(x, num_groups, weight, bias, split, eps)
+    return _GroupNormOutput.apply(x, num_groups, weight, bias, split, eps, torch.is_grad_enabled())
 
 
 __all__ = ["_GroupNorm", "group_norm", "partial_sqdev", "partial_sum"]

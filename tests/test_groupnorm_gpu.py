@@ -183,3 +183,32 @@ def test_group_norm_without_x_norm(case, dev):
     y0 = jgn.group_norm(x0, G, w, b, (others,))
     g0, = torch.autograd.grad(y0, x0, g.chunk(P, 2)[0])
     assert not others.parts and rel_l2(y0, want.chunk(P, 2)[0]) < tol and rel_l2(g0, grads[0].chunk(P, 2)[0]) < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(2, 8, 16, 24), (1, 6, 7, 9)], ids=str)  # rows on and off the 16-byte grid
+@pytest.mark.parametrize("sharded", [False, True])
+def test_input_changed_in_place_before_the_backward(shape, dtype, sharded, dev):
+    """``x += group_norm(x)`` and an activation in place on the result: the backward has what it needs of its own."""
+    torch.manual_seed(5)
+    leaf = torch.randn(*shape, device=dev).to(dtype).requires_grad_()
+    w = (1 + 0.2 * torch.randn(shape[1], device=dev)).to(dtype).requires_grad_()
+    b = (0.2 * torch.randn(shape[1], device=dev)).to(dtype).requires_grad_()
+    g = torch.randn(*shape, device=dev).to(dtype)
+
+    class Alone:  # a spatial group whose other ranks hold nothing
+        def size(self):
+            return 2
+
+        def all_reduce(self, t, op):
+            pass
+
+    x = leaf * 1
+    y = jgn.group_norm(x, 2, w, b, (Alone(),) if sharded else ())
+    x += y
+    grads = torch.autograd.grad(x, (leaf, w, b), g)
+    ref = [t.detach().double().requires_grad_() for t in (leaf, w, b)]
+    want = ref[0] + torch.nn.functional.group_norm(ref[0], 2, ref[1], ref[2], 1e-5)
+    for a, r in zip(grads, torch.autograd.grad(want, ref, g.double())):
+        assert rel_l2(a, r) < max(TOL[dtype], 2e-5)
+    assert rel_l2(x, want) < TOL[dtype]
