@@ -152,6 +152,11 @@ __device__ __forceinline__ u32x4 map8(u32x4 y, u32x4 r, F f) {
 __device__ __forceinline__ void dma_1k(const void* base, uint32_t lane_off, uint32_t lds_dst) {
   asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(base), "s"(lds_dst));
 }
+// The same for operands of 2^32 bytes and more: 64-bit offsets, added to the base lane by lane.
+__device__ __forceinline__ void dma_1k(const void* base, uint64_t lane_off, uint32_t lds_dst) {
+  const char* at = static_cast<const char*>(base) + lane_off;
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(at), "s"(lds_dst));
+}
 __device__ __forceinline__ uint32_t lds_address(const unsigned char* p) {
   typedef __attribute__((address_space(3))) unsigned char* lds_bytes;
   return (uint32_t)(uintptr_t)((lds_bytes)p);
@@ -418,21 +423,23 @@ struct TnShape {
 };
 
 // Tokens r, r + step, ... of an operand as byte offsets; heads: (b * H * S + s) * D, row-major: r * ld.
+// OFF: uint32_t, or uint64_t where an operand has 2^32 bytes or more.
+template <typename OFF>
 struct TokenWalk {
-  uint32_t off;      // bytes
-  int s, S;          // position in the batch entry and its length
-  uint32_t row, jump;  // bytes between tokens of an entry; extra bytes from the end of an entry to the next one
+  OFF off;         // bytes
+  int s, S;        // position in the batch entry and its length
+  OFF row, jump;   // bytes between tokens of an entry; extra bytes from the end of an entry to the next one
   __device__ __forceinline__ void start(const Map& m, long long r) {
-    row = (uint32_t)(m.heads ? m.D : m.ld) * 2u;
+    row = (OFF)(m.heads ? m.D : m.ld) * 2u;
     S = m.heads ? m.S : 0x7fffffff;
-    jump = m.heads ? (uint32_t)(m.H - 1) * (uint32_t)m.S * row : 0u;
+    jump = m.heads ? (OFF)(m.H - 1) * (OFF)m.S * row : 0u;
     const long long b = m.heads ? r / m.S : 0;
-    s = (int)(r - b * S);
-    off = (uint32_t)(row_part(m, r) * 2);
+    s = m.heads ? (int)(r - b * S) : 0;
+    off = (OFF)(row_part(m, r) * 2);
   }
   __device__ __forceinline__ void advance(int by) {
     s += by;
-    off += (uint32_t)by * row;
+    off += (OFF)by * row;
     while (s >= S) {  // at most once where an entry is longer than the step
       s -= S;
       off += jump;
@@ -447,7 +454,9 @@ struct TokenWalk {
 // instruction transposes: with its reduction 72 us for 32768 tokens, 1536 x 512 (101 us with both and a round more), 1132 us for
 // 8192 x 8192 x 8192 (1294). A batch entry may be of any length: the octet-wise staging took multiples of 8 tokens
 // only and left the rest to the FMA kernel (5 x 590 tokens, 896 features, qkv and output projection: 2247 -> 250 us). The bias gradient is one more matrix instruction with ones, in the first column of tiles.
-template <int IM, int JN, int WM, int WN>
+// OFF as in TokenWalk: 64-bit offsets from 2^32 bytes an operand on, at the same rate (2048 x 512 over 2^20 tokens 2.44 ms,
+// 2040 x 512 with 32-bit ones 2.48; the FMA kernel, which the larger one would else fall to, 238 ms).
+template <int IM, int JN, int WM, int WN, typename OFF>
 __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_kernel(TnParams p) {
   typedef TnShape<IM, JN, WM, WN> SH;
   constexpr int T = SH::T, ROWB = SH::ROWB;
@@ -476,9 +485,9 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
   const int my_row = wave * SH::RPI + lane / SH::CPR;
   const int chunk = (lane % SH::CPR) ^ ((my_row & 3) << 2);  // JROWS is a multiple of 4: the same for every j
   // a chunk past the last feature repeats the last one and is dropped
-  const uint32_t gf = (uint32_t)(feat_part(p.gm, min(n0 + chunk * 8, p.N - 8)) * 2);
-  const uint32_t xf = (uint32_t)(feat_part(p.xm, min(c0 + chunk * 8, p.C - 8)) * 2);
-  TokenWalk gw, xw;
+  const OFF gf = (OFF)(feat_part(p.gm, min(n0 + chunk * 8, p.N - 8)) * 2);
+  const OFF xf = (OFF)(feat_part(p.xm, min(c0 + chunk * 8, p.C - 8)) * 2);
+  TokenWalk<OFF> gw, xw;
   gw.start(p.gm, min(r_first + my_row, p.rows - 1));
   xw.start(p.xm, min(r_first + my_row, p.rows - 1));
   const uint32_t lds_g = lds_address(smem) + wave_u * 1024;
@@ -486,7 +495,7 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
     const long long left = p.rows - (r_first + (long long)st * BR);
     const uint32_t dst = lds_g + buf * SH::STAGE;
     if (left >= BR) {  // wave-uniform
-      TokenWalk a = gw, b = xw;
+      TokenWalk<OFF> a = gw, b = xw;
 #pragma unroll
       for (int j = 0; j < SH::DMA; ++j) {
         dma_1k(p.g, a.off + gf, dst + j * SH::WAVES * 1024);
@@ -500,14 +509,14 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
 #pragma unroll
       for (int j = 0; j < SH::DMA; ++j) {
         const long long r = min(r_first + (long long)st * BR + j * SH::JROWS + my_row, p.rows - 1);
-        dma_1k(p.g, (uint32_t)(row_part(p.gm, r) * 2) + gf, dst + j * SH::WAVES * 1024);
-        dma_1k(p.x, (uint32_t)(row_part(p.xm, r) * 2) + xf, dst + SH::OP + j * SH::WAVES * 1024);
+        dma_1k(p.g, (OFF)(row_part(p.gm, r) * 2) + gf, dst + j * SH::WAVES * 1024);
+        dma_1k(p.x, (OFF)(row_part(p.xm, r) * 2) + xf, dst + SH::OP + j * SH::WAVES * 1024);
       }
     }
   };
   static_assert(SH::DMA * SH::JROWS == BR, "the walkers stand at the next stage after their transfers");
   auto clear_tail = [&](int st, int buf) {
-    const int left = (int)(p.rows - (r_first + (long long)st * BR));
+    const long long left = p.rows - (r_first + (long long)st * BR);
     if (left >= BR) return;
     u32x4* at = reinterpret_cast<u32x4*>(smem + buf * SH::STAGE + wave * 1024 + lane * 16);
 #pragma unroll
@@ -910,12 +919,12 @@ int tn_splits(long long rows, int n, int c) {
   return (int)want;
 }
 
-template <int IM, int JN, int WM, int WN>
+template <int IM, int JN, int WM, int WN, typename OFF>
 int launch_tn(TnParams& p, int splits, hipStream_t s, const char* who) {
   typedef TnShape<IM, JN, WM, WN> SH;
   p.tiles_c = jg::cdiv(p.C, SH::T);
   p.tiles = jg::cdiv(p.N, SH::T) * p.tiles_c;
-  void (*kern)(TnParams) = &proj_tn_kernel<IM, JN, WM, WN>;
+  void (*kern)(TnParams) = &proj_tn_kernel<IM, JN, WM, WN, OFF>;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS) != hipSuccess)
     JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, SH::LDS);
   kern<<<(unsigned)p.tiles * (unsigned)splits, SH::THREADS, SH::LDS, s>>>(p);
@@ -1069,8 +1078,7 @@ int jg_proj_tn(void* gw, void* gb, const void* g, const void* x, int dtype, int 
   rc = make_map(&xm, x_heads, c, rows, B, H, S, D, who, "input");
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool fast = dtype == JG_BF16 && map_vec_ok(gm, n) && map_vec_ok(xm, c) && aligned16(g) && aligned16(x) &&
-                    (unsigned long long)rows * n < (1ull << 31) && (unsigned long long)rows * c < (1ull << 31);
+  const bool fast = dtype == JG_BF16 && map_vec_ok(gm, n) && map_vec_ok(xm, c) && aligned16(g) && aligned16(x);
   if (!fast) {
     GenParams gp;
     gp.p = g; gp.q = x; gp.bias = nullptr; gp.out = gw;
@@ -1103,7 +1111,11 @@ int jg_proj_tn(void* gw, void* gb, const void* g, const void* x, int dtype, int 
   p.stages_per_split = (int)((stages + splits - 1) / splits);
   p.part = static_cast<float*>(workspace);
   p.bias_part = gb != nullptr ? p.part + (size_t)splits * n * c : nullptr;
-  rc = tn_tile(rows, n, c) == 256 ? launch_tn<4, 2, 2, 4>(p, splits, s, who) : launch_tn<2, 2, 2, 2>(p, splits, s, who);
+  const bool far = (unsigned long long)rows * (n > c ? n : c) >= (1ull << 31);
+  if (tn_tile(rows, n, c) == 256)
+    rc = far ? launch_tn<4, 2, 2, 4, uint64_t>(p, splits, s, who) : launch_tn<4, 2, 2, 4, uint32_t>(p, splits, s, who);
+  else
+    rc = far ? launch_tn<2, 2, 2, 2, uint64_t>(p, splits, s, who) : launch_tn<2, 2, 2, 2, uint32_t>(p, splits, s, who);
   if (rc) return rc;
   ReduceArgs ra{};
   ra.out_w = gw;

@@ -79,3 +79,14 @@ def test_misaligned_chunks_are_refused_without_a_gpu(which, d):
         rc = lib.jg_attn_bwd_chunks(p["dq"], one("dk"), one("dv"), p["dout"], p["q"], one("k"), one("v"), 1, p["out"], p["lse"], 2,
                                     sq, sk, d, 0.125, bf16, p["ws"], 1 << 20, None)
         assert rc == -2 and b"aligned" in lib.jg_last_error()
+
+
+def test_weight_gradient_of_large_operands_keeps_its_kernel_without_a_gpu():
+    """jg_proj_tn on bf16 operands of 2^32 bytes and more: the matrix-core kernel, which asks for its workspace (the
+    one-product-at-a-time kernel needs none)."""
+    lib = jigsaw_amd.load()
+    bf16, at = _lib.dtype_code(torch.bfloat16), ctypes.c_void_p(0x1000)
+    for rows, n, c in ((1 << 20, 2048, 64), (1 << 20, 64, 2048), (1 << 22, 1536, 512), (1 << 32, 8, 8)):
+        assert lib.jg_proj_tn_workspace(rows, n, c) > 0
+        rc = lib.jg_proj_tn(at, at, at, at, bf16, bf16, rows, n, c, 0, 0, 1, 1, 1, 1, None, 0, None)
+        assert rc == -4 and b"workspace" in lib.jg_last_error(), (rc, rows, n, c)

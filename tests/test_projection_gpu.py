@@ -293,3 +293,33 @@ def test_gemm_tiles_with_remainders(b, s, c, n_out, heads, dev):
         assert rel_l2(got[0].reshape(-1, c), g2 @ w.float()) < 1e-2
         assert rel_l2(got[1], g2.t() @ x2) < 1e-2
         assert rel_l2(got[2], g2.sum(0)) < 1e-2
+
+
+@pytest.mark.parametrize("heads", [False, True])
+@pytest.mark.parametrize("rows,n,c", [((1 << 20) + 37, 2048, 64), (8 * 90001, 3072, 256)], ids=str)
+def test_weight_gradient_of_operands_beyond_four_gigabytes(rows, n, c, heads, dev):
+    """Byte offsets past 2^32, row-major and in the heads layout, both tile sizes, a ragged last stage: every token counts
+    once. The operands hold small whole numbers, so fp32 sums in any order are exact."""
+    torch.manual_seed(n)
+    B, D = (8, 64) if rows % 8 == 0 else (1, 64)
+    S, t = rows // B, 3 if n % 3 == 0 else 1
+    H = n // (t * D)
+    g = torch.randint(-2, 3, (t, B, H, S, D) if heads else (rows, n), device=dev, dtype=torch.int8).to(torch.bfloat16)
+    x = torch.randint(-1, 2, (rows, c), device=dev, dtype=torch.int8).to(torch.bfloat16)
+    assert g.numel() >= 1 << 31
+    gw, gb = jp._tn(g, x, rows, n, c, heads, False, (B, H, S, D), True, torch.float32)
+    want_w, want_b = torch.zeros(n, c, device=dev), torch.zeros(n, device=dev)
+    if heads:
+        for i in range(t):
+            for b in range(B):
+                part = g[i, b].float()  # (H, S, D)
+                xb = x[b * S:(b + 1) * S].float()
+                at = slice(i * H * D, (i + 1) * H * D)
+                want_w[at] += torch.cat([part[h].t() @ xb for h in range(H)])
+                want_b[at] += part.sum(1).flatten()
+    else:
+        for r in range(0, rows, 1 << 17):
+            part = g[r:r + (1 << 17)].float()
+            want_w += part.t() @ x[r:r + (1 << 17)].float()
+            want_b += part.sum(0)
+    assert torch.equal(gw, want_w) and torch.equal(gb, want_b)
