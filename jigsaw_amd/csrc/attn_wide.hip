@@ -787,24 +787,11 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
     }
 }
 
-int cu_count() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-      cus = n;
-    else
-      cus = 256;
-  }
-  return cus;
-}
-
 // Groups per workgroup. A launch that leaves CUs without a workgroup splits the streamed side over more wavefronts
 // of one: up to 4 groups where the registers of 16 wavefronts hold the state (forward, D <= 64), else 2.
 int split_of(long long workgroups, int most) {
   int ks = 1;
-  while (ks < most && workgroups * ks < cu_count()) ks *= 2;
+  while (ks < most && workgroups * ks < jg::cu_count()) ks *= 2;
   return ks;
 }
 
@@ -851,7 +838,7 @@ int launch_bwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_
   if constexpr (D <= (EXACT ? 64 : 96)) {
     if (split_of(dkv_workgroups, 2) == 2)
       return launch(&attn_wide_dkv_kernel<D, F16, 0, 2, EXACT>, dkv_grid, 2 * GROUP, 2 * DKV_LDS, tab, a, s, who);
-  } else if (EXACT || dkv_workgroups > cu_count()) {
+  } else if (EXACT || dkv_workgroups > jg::cu_count()) {
     rc = launch(&attn_wide_dkv_kernel<D, F16, 1, 1, EXACT>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
     if (rc != JG_OK) return rc;
     return launch(&attn_wide_dkv_kernel<D, F16, 2, 1, EXACT>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);

@@ -1230,17 +1230,6 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
 }
 
 // ----------------------------------------------------------------- host side
-int cu_count() {
-  static int cached = 0;
-  if (cached) return cached;
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-    n = 256;
-  cached = n;
-  return n;
-}
-
 // How a problem maps onto the kernel: produced channels in tiles of MT (M padded up to a
 // multiple of 32 with zero weight rows), contraction steps of 16 channels in groups of wc16
 // steps whose weights fit LDS beside the two input stages.
@@ -1323,7 +1312,7 @@ size_t conv_ws_bytes(int split, int KD, int C, int M, size_t x_elements, bool ph
 // latency) on every compute unit, one after the other. 64 -> 128 channels of 4 x 256 x 256 at stride 2 forward 32.7 -> 27.2 us;
 // 96 -> 96 of 4 x 128 x 256 input gradient 62 -> 54 us, 64 -> 128 of 8 x 512 x 512 forward 320 -> 305 us.
 int workgroups_for(long long tiles, int mtiles) {
-  const long long cus = cu_count() / 8 > 0 ? cu_count() / 8 : 1;  // of an XCD
+  const long long cus = jg::cu_count() / 8 > 0 ? jg::cu_count() / 8 : 1;  // of an XCD
   const long long share = (tiles + 7) / 8;                        // tiles of an XCD
   const long long all = share < cus ? share : cus;
   if (mtiles > 1 && mtiles <= cus) {

@@ -864,17 +864,6 @@ __global__ __launch_bounds__(256) void wgrad_combine_parts_kernel(float* __restr
   gw[idx] = sum;
 }
 
-int cu_count() {
-  static int cached = 0;
-  if (cached) return cached;
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-    n = 256;
-  cached = n;
-  return n;
-}
-
 int stage_columns(const ConvGeom& g) { return g.s[2] == 2 ? Stage<2>::SW : Stage<1>::SW; }
 long long stage_count(const ConvGeom& g) {
   const int sw = stage_columns(g);
@@ -931,7 +920,7 @@ Plan plan_of(const ConvGeom& g, int parts) {
   const long long stages = stage_count(g);
   const double blocks = (double)p.blocks(), bytes = (double)p.partial() * sizeof(float);
   const double best = sqrt((double)stages * blocks * 4.0e6 / bytes);
-  const double most = cu_count() * (p.cgb * p.cxb == 1 ? 2.0 : 1.0);
+  const double most = jg::cu_count() * (p.cgb * p.cxb == 1 ? 2.0 : 1.0);
   long long n = (long long)((best < most ? best : most) / blocks);
   if (n >= 8) n = n / 8 * 8;
   if (n > stages) n = stages;

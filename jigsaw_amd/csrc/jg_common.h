@@ -58,4 +58,14 @@ __host__ __device__ static inline uint16_t f32_to_bf16(float f) {
 
 static inline int cdiv(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
+// Compute units of the device (of a partition of it, where the device is one): what the host-side rules that fill the
+// chip count with. Asked once; 256, a whole MI355X, where there is no device to ask (sizes of workspaces on the CPU).
+inline int cu_count() {
+  static const int count = [] {
+    int dev = 0, n = 0;
+    return hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
+  }();
+  return count;
+}
+
 }  // namespace jg

@@ -387,7 +387,7 @@ int launch_nt(NtParams& p, hipStream_t s, const char* who) {
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS) != hipSuccess)
     JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, SH::LDS);
   // as many workgroups as fit at once (a multiple of 8: one share per XCD)
-  const long long fit = 256 * (160 * 1024 / SH::LDS);
+  const long long fit = (long long)jg::cu_count() * (160 * 1024 / SH::LDS);
   const unsigned grid = (unsigned)(((tiles < fit ? tiles : fit) + 7) / 8 * 8);
   kern<<<grid, SH::THREADS, SH::LDS, s>>>(p);
   JG_CHECK_LAUNCH(who);
@@ -884,22 +884,22 @@ int tn_tile(long long rows, int n, int c) {
   if (n < 256 || c < 256) return 128;
   const long long tiles = (long long)jg::cdiv(n, 256) * jg::cdiv(c, 256);
   const long long most = tn_stages(rows) / 8;
-  return tiles * (most < 1 ? 1 : most < TN_MOST_SPLITS ? most : TN_MOST_SPLITS) >= 192 ? 256 : 128;
+  return tiles * (most < 1 ? 1 : most < TN_MOST_SPLITS ? most : TN_MOST_SPLITS) >= jg::cu_count() * 3 / 4 ? 256 : 128;
 }
 // Token ranges the contraction is cut into so that the tiles fill the chip.
 int tn_splits(long long rows, int n, int c) {
   const int t = tn_tile(rows, n, c);
-  const long long tiles = (long long)jg::cdiv(n, t) * jg::cdiv(c, t), stages = tn_stages(rows);
+  const long long tiles = (long long)jg::cdiv(n, t) * jg::cdiv(c, t), stages = tn_stages(rows), cus = jg::cu_count();
   if (t == 256) {
-    // One workgroup fits a compute unit, so a few more than 256 of them cost a second round: 12 tiles in 22 splits
+    // One workgroup fits a compute unit, so a few more than these (256) cost a second round: 12 tiles in 22 splits
     // (1536 x 512 over 32768 tokens) took 88 us, in 21 splits 72. The number of splits with the least of: rounds of
-    // 256 times the stages of a split (1.7 us each, 5 us around them), and the partials, written and read back at about
+    // workgroups times the stages of a split (1.7 us each, 5 us around them), and the partials, written and read back at about
     // 6 TB/s. 3072 x 1024 over 8192 tokens 102 -> 74 us (6 -> 5 splits), 2112 x 704 over 20000 125 -> 91 us (10 -> 9),
     // 512 x 512 over 32768 44 -> 41 us (64 -> 47).
     int best = 1;
     double least = 0.0;
     for (int k = 1; k <= TN_MOST_SPLITS && (k == 1 || k <= stages / 8); ++k) {
-      const double rounds = (double)((tiles * k + 255) / 256), walk = (double)((stages + k - 1) / k);
+      const double rounds = (double)((tiles * k + cus - 1) / cus), walk = (double)((stages + k - 1) / k);
       const double us = rounds * (walk * 1.7 + 5.0) + k * (double)n * c * 8.0 / 6.0e6;
       if (k == 1 || us < least) {
         least = us;
@@ -911,8 +911,8 @@ int tn_splits(long long rows, int n, int c) {
   // 128: two workgroups a compute unit, two rounds of them; at most 64 splits, but with one to three tiles as many
   // as put a workgroup on every compute unit: a compute unit streams its operands at some 20 GB/s, so 64 workgroups
   // leave three quarters of the memory system idle (128 x 128 over 65536 tokens: 23 -> 13 us, the reduction 5 -> 6 us)
-  const long long cap = tiles * TN_MOST_SPLITS >= 256 ? TN_MOST_SPLITS : 256 / tiles;
-  long long want = (1024 + tiles - 1) / tiles;
+  const long long cap = tiles * TN_MOST_SPLITS >= cus ? TN_MOST_SPLITS : cus / tiles;
+  long long want = (4 * cus + tiles - 1) / tiles;
   if (want > stages / (cap > TN_MOST_SPLITS ? 4 : 8)) want = stages / (cap > TN_MOST_SPLITS ? 4 : 8);
   if (want < 1) want = 1;
   if (want > cap) want = cap;
@@ -990,9 +990,9 @@ static int proj_nt_common(const char* who, void* out, void* aux, int epi, const 
   const long long big_tiles = (long long)jg::cdiv(rows, 256) * jg::cdiv(n_out, 256);
   // the 256-wide tile only where its last column of tiles is more than half full
   const int waste = jg::cdiv(n_out, 256) * 256 - n_out;
-  if (big_tiles >= 256 && waste < 128) return launch_nt<4, 2, 2, 4>(p, s, who);
+  if (big_tiles >= jg::cu_count() && waste < 128) return launch_nt<4, 2, 2, 4>(p, s, who);
   // 64 x 64 where 128 x 128 tiles would leave most of the chip idle (468 tokens, 704 -> 2112: 7.9 us, 13.1 before)
-  if ((long long)jg::cdiv(rows, 128) * jg::cdiv(n_out, 128) < 128) return launch_nt<1, 1, 2, 2>(p, s, who);
+  if ((long long)jg::cdiv(rows, 128) * jg::cdiv(n_out, 128) < jg::cu_count() / 2) return launch_nt<1, 1, 2, 2>(p, s, who);
   return launch_nt<2, 2, 2, 2>(p, s, who);
 }
 
