@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
+import warnings
 from ctypes import POINTER, c_char_p, c_double, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
@@ -353,16 +354,19 @@ def load() -> ctypes.CDLL:
 
 
 def host():
-    """The native host module (``csrc/host.cpp``), imported once."""
+    """The native host module (``csrc/host.cpp``), imported once; ``None`` where it is not built or does not load, which a
+    warning says once: the Python routes then do its work, with the same kernels and results and more host time."""
     global _host
     if _host is None:
         load()
         try:
             from . import _host as module
         except ImportError as e:
-            raise LibraryMissing(f"jigsaw_amd/_host.so is not built or does not load ({e}). Run `python -m jigsaw_amd.build`.") from e
+            module = False
+            warnings.warn(f"jigsaw_amd/_host.so is not built or does not load ({e}): convolutions take the slower Python route. "
+                          "Run `python -m jigsaw_amd.build`.", RuntimeWarning, stacklevel=2)
         _host = module
-    return _host
+    return _host or None
 
 
 def abi_version() -> int:

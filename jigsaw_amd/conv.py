@@ -968,8 +968,10 @@ def _frame_decision(config, x, geom: HaloGeometry, weight_shape, kwargs):
 @lru_cache(maxsize=256)
 def _step(x_shape, dtype, w_shape, stride, padding, dilation, ranks, sizes, groups: int, fused_fold: bool):
     """The native host plan (``csrc/host.cpp``) of a layer on a tile, or ``None`` where the Python route below runs it:
-    layers that are re-shaped before they reach the kernels, spans that the strips do not cover."""
-    n = len(w_shape) - 2
+    layers that are re-shaped before they reach the kernels, spans that the strips do not cover, no host module."""
+    n, host = len(w_shape) - 2, _lib.host()
+    if host is None:
+        return None
     if dtype not in _lib._DTYPES or len(x_shape) != n + 2:
         return None
     if not spans_fit_the_strips(x_shape[-n:], w_shape[-n:], stride, padding, dilation, sizes):
@@ -984,7 +986,7 @@ def _step(x_shape, dtype, w_shape, stride, padding, dilation, ranks, sizes, grou
     rows = {verb: [(o, i, lead + extent) for o, i, extent in rows] for verb, rows in geom._extents.items()}
     sent = lambda verb: [row for row in rows[verb] if row[0] in present]  # noqa: E731
     address = lambda c: ctypes.addressof(c)  # noqa: E731
-    return _lib.host().Step(
+    return host.Step(
         tuple(x_shape), lead + geom.padded, launches[0].shape, tuple(w_shape), dtype.itemsize, _lib.dtype_code(dtype),
         address(geom.c_geom(planes)), address(geom.theirs().c_geom(planes)), geom.same_on_every_rank, address(launches[0].desc),
         [launch.nbytes for launch in launches], rows["assemble"], rows["fold"], sent("pack_fwd"), sent("pack_bwd"),

@@ -1,0 +1,89 @@
+"""The native host module of the distributed convolution beside the Python route it shortens."""
+
+import itertools
+import sys
+
+import pytest
+import torch
+
+from jigsaw_amd import _lib
+from jigsaw_amd import conv as jc
+from jigsaw_amd.halo import HaloGeometry
+
+
+def test_a_host_module_that_does_not_load_leaves_the_python_route(monkeypatch):
+    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.setitem(sys.modules, "jigsaw_amd._host", None)  # import raises ImportError
+    monkeypatch.delattr("jigsaw_amd._host", raising=False)
+    jc._step.cache_clear()
+    try:
+        with pytest.warns(RuntimeWarning, match="_host.so"):
+            step = jc._step((1, 4, 8, 8), torch.float32, (4, 4, 3, 3), (1, 1), (1, 1), (1, 1), (0, 0), (2, 2), 1, True)
+        assert step is None and _lib.host() is None  # said once
+    finally:
+        jc._step.cache_clear()
+
+
+class _Held:
+    """The halo exchange of a rank whose neighbours' strips are here already."""
+
+    def __init__(self, fwd, bwd):
+        self.fwd, self.bwd, self.sent = fwd, bwd, []
+
+    def forward(self, send):
+        self.sent.append(send)
+        return self.fwd
+
+    def backward(self, send):
+        self.sent.append(send)
+        return self.bwd
+
+
+ROUTE_CASES = [
+    # size, batch, c_in, c_out, kernel, stride, padding, mesh, rank, groups, dtype, bias
+    ((16, 24), 2, 3, 16, 3, 1, 1, 3, 1, 1, torch.float32, True),
+    ((16, 64), 2, 64, 64, 3, 1, 1, 3, 1, 1, torch.bfloat16, True),    # the fused fold
+    ((17, 23), 1, 40, 72, 3, 1, 1, 2, 0, 1, torch.bfloat16, True),    # the fold of its own
+    ((16, 32), 2, 32, 64, 3, 2, 1, 2, 1, 1, torch.bfloat16, False),   # stride 2
+    ((12, 16), 1, 4, 6, 3, 1, 0, 2, 1, 1, torch.float16, True),       # halos that differ from rank to rank
+    ((6, 8, 16), 1, 32, 32, 3, 1, 1, 3, 1, 1, torch.bfloat16, True),
+    ((8, 12), 2, 6, 9, 3, 1, 1, 3, 1, 3, torch.float32, True),        # grouped
+    ((8, 12), 2, 6, 9, 3, 1, 1, 1, 0, 1, torch.float32, True),        # nothing to exchange
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ROUTE_CASES, ids=lambda c: f"{c[2]}to{c[3]}_{'x'.join(map(str, c[0]))}_s{c[5]}_mesh{c[7]}")
+def test_native_and_python_route_of_a_step_agree_bit_for_bit(case, monkeypatch):
+    size, batch, ci, co, k, s, p, mesh, rank, cgroups, dtype, bias = case
+    dev, n = torch.device("cuda:0"), len(size)
+    torch.manual_seed(3)
+    kernel, stride, padding, dilation = (k,) * n, (s,) * n, (p,) * n, (1,) * n
+    geom = HaloGeometry.for_conv(size, kernel, stride, padding, dilation, (rank,) * n, (mesh,) * n)
+    mk = lambda *shape: torch.randn(*shape, device=dev).to(dtype)  # noqa: E731
+    present = [o for o in itertools.product((-1, 0, 1), repeat=n) if any(o) and all(0 <= rank + v < mesh for v in o)]
+    strips = [{o: mk(batch, ci, *geom.strip_extent(o, verb)) for o in present} for verb in ("assemble", "fold")]
+    x, w = mk(batch, ci, *size).requires_grad_(), mk(co, ci // cgroups, *kernel).requires_grad_()
+    b = mk(co).requires_grad_() if bias else None
+    spatial = tuple(jc.TileGroup(mesh, rank) for _ in size)
+    made = []
+    step_for = jc._step_for
+
+    def run(native):
+        def chosen(*a):
+            made.append(step_for(*a))
+            return made[-1] if native else None
+
+        monkeypatch.setattr(jc, "_step_for", chosen)
+        held = _Held(*strips)
+        y, x_aug = jc._ConvNd.apply(x, w, b, stride, padding, dilation, spatial, None,
+                                    jc.HipConvNdConfig.for_rank(n, b, held, groups=cgroups))
+        torch.manual_seed(4)
+        grads = torch.autograd.grad(y, [t for t in (x, w, b) if t is not None], mk(*y.shape))
+        return [y, x_aug, *grads, *(d[o] for d in held.sent for o in sorted(d))]
+
+    native, python = run(True), run(False)
+    assert all(m is not None for m in made), "the native route does not take this case"
+    assert len(native) == len(python)
+    for a, c in zip(native, python):
+        assert a.shape == c.shape and a.dtype == c.dtype and torch.equal(a, c)
