@@ -103,7 +103,8 @@ def _bias_args(bias, batch, sq, sk):
 # The 16-bit matrix-core kernels take any lengths and any head size that is a multiple of 8 up to
 # 128, the fp32 ones any lengths at three head sizes, the one-thread-per-row kernels (bias, more
 # batch entries than a grid dimension holds) a few head sizes. Other head sizes get zero columns:
-# they add nothing to the scores and give zero output columns, which are dropped.
+# they add nothing to the scores and give zero output columns, which are dropped. Narrow bf16 heads on
+# long sequences get them too, for the faster kernels of 64 columns (_as_64_columns).
 # --------------------------------------------------------------------------- #
 _KERNEL_HEAD_SIZES = (8, 16, 32, 64, 96, 128)
 _F32_MFMA_HEAD_SIZES = (32, 64, 128)
@@ -125,9 +126,26 @@ def _kernel_head_size(d: int, dtype=None, has_bias: bool = False) -> int:
     return next((n for n in sizes if n >= d), d)
 
 
+def _as_64_columns(q, k, chunks: int = 1) -> bool:
+    """Whether bf16 heads of fewer than 64 columns against ``chunks`` chunks like ``k`` are better off with zero columns
+    up to 64, copies there and back included, on the kernels of that size, which stream their tiles straight into LDS and keep eight
+    wavefronts busy a workgroup. Forward / backward, us, own width and as 64 columns: 8 heads x 4096 x 4096 keys, 16 columns
+    119/306 and 69/169, 48 columns 131/333 and 72/178; 32 heads 238/647 and 197/514, 276/754 and 206/560; but 32 heads x 2048 x 2048
+    70/173 and 87/182, 80/204 and 91/196, and 128 heads x 1024 x 2 chunks of 1024 keys 123/329 and 149/374. A width of 32 is a
+    kernel's own, and worth leaving only where its four wavefronts a workgroup leave compute units idle: 8 heads x 4096 x
+    4096 keys 93/237 and 68/173, 16 heads 106/260 and 121/288."""
+    d, sq, keys = q.shape[-1], q.shape[-2], k.shape[-2] * chunks
+    if q.dtype != torch.bfloat16 or d >= 64 or sq < 2048 or keys < 4096:
+        return False
+    rows = math.prod(q.shape[:-1])
+    return rows * keys >= 1 << 27 and sq >= 4096 and rows <= 1 << 15 if 24 < d <= 32 else True
+
+
 def _padded_head_size(q, k, bias) -> int:
     d = q.shape[-1]
-    return (d + 7) // 8 * 8 if _mfma16(q, k, bias) else _kernel_head_size(d, q.dtype, bias is not None)
+    if not _mfma16(q, k, bias):
+        return _kernel_head_size(d, q.dtype, bias is not None)
+    return 64 if _as_64_columns(q, k) else (d + 7) // 8 * 8
 
 
 def _pad_last(t: torch.Tensor, to: int) -> torch.Tensor:
@@ -240,6 +258,8 @@ def _fused_ok(q, k) -> bool:
     d = q.shape[-1]
     if any(t.data_ptr() % 16 for t in (q, k)):
         return False
+    if _as_64_columns(q, k):  # the merge is a kernel of its own then, 32 heads x 4096 x 4096 keys of 16 columns 187 us, fused 239
+        return False
     return d in _F32_MFMA_HEAD_SIZES if q.dtype == torch.float32 else d % 8 == 0 and _mfma16(q, k)
 
 
@@ -293,10 +313,19 @@ def _pointers(tensors) -> ctypes.Array:
     return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
 
 
+def _chunks_as_64_columns(chunks) -> list:
+    """The chunks with zero columns up to 64: three launches for all of them."""
+    return list(_pad_last(torch.stack(tuple(chunks)), 64).unbind(0))
+
+
 def _resident_forward(q, k_chunks, v_chunks, scale):
     """``(out, lse)`` over resident chunks in ONE launch (``jg_attn_fwd_chunks``), ``None`` where that does not cover them."""
     if not k_chunks or not _resident(q, k_chunks, v_chunks):
         return None
+    if _as_64_columns(q, k_chunks[0], len(k_chunks)):
+        kv = _chunks_as_64_columns(t.to(q.dtype) for t in (*k_chunks, *v_chunks))
+        out, lse = _resident_forward(_pad_last(q, 64), kv[:len(k_chunks)], kv[len(k_chunks):], scale)
+        return out[..., :q.shape[-1]].contiguous(), lse
     q = _dense(q)
     ks, vs = [_dense(t.to(q.dtype)) for t in k_chunks], [_dense(t.to(q.dtype)) for t in v_chunks]
     batch, sq, d = _flat(q)
@@ -317,6 +346,18 @@ def _resident_backward(dout, q, out, lse, k_chunks, v_chunks, scale):
     if not k_chunks or not _resident(q, k_chunks, v_chunks):
         return None
     _lib.require_gpu(dout, q, out, lse)
+    if _as_64_columns(q, k_chunks[0], len(k_chunks)):
+        d, P = q.shape[-1], len(k_chunks)
+        kv = _chunks_as_64_columns(t.to(q.dtype) for t in (*k_chunks, *v_chunks))
+        dq, dkv = _backward_over(*(_pad_last(t.to(q.dtype), 64) for t in (dout, q, out)), lse, kv[:P], kv[P:], scale)
+        dkv = dkv[..., :d].contiguous()
+        return dq[..., :d].contiguous(), list(dkv[0].unbind(0)), list(dkv[1].unbind(0))
+    dq, dkv = _backward_over(dout, q, out, lse, k_chunks, v_chunks, scale)
+    return dq, list(dkv[0].unbind(0)), list(dkv[1].unbind(0))
+
+
+def _backward_over(dout, q, out, lse, k_chunks, v_chunks, scale):
+    """``(dq, dkv)`` of ``jg_attn_bwd_chunks``; ``dkv[0][j]``, ``dkv[1][j]`` are chunk j's dK and dV (one allocation)."""
     dout, out, q = _dense(dout.to(q.dtype)), _dense(out.to(q.dtype)), _dense(q)
     lse = lse.to(torch.float32).contiguous()
     ks, vs = [_dense(t.to(q.dtype)) for t in k_chunks], [_dense(t.to(q.dtype)) for t in v_chunks]
@@ -324,7 +365,6 @@ def _resident_backward(dout, q, out, lse, k_chunks, v_chunks, scale):
     batch, sq, d = _flat(q)
     sk = int(ks[0].shape[-2])
     dq = torch.empty_like(q)
-    # one allocation for all partials: chunk j's dK / dV are views of it
     dkv = torch.empty((2, P) + tuple(ks[0].shape), dtype=q.dtype, device=q.device)
     dks, dvs = list(dkv[0].unbind(0)), list(dkv[1].unbind(0))
     lib = _lib.load()
@@ -336,7 +376,7 @@ def _resident_backward(dout, q, out, lse, k_chunks, v_chunks, scale):
         _lib.stream_ptr(q.device),
     )
     _lib.check(rc, "jg_attn_bwd_chunks")
-    return dq, dks, dvs
+    return dq, dkv
 
 
 def backward_chunks(dout, q, out, lse, k_chunks, v_chunks, scale):

@@ -847,7 +847,8 @@ int launch_bwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_
   return JG_OK;
 }
 
-// f(D constant, F16 constant) for the narrowest kernel that holds the head
+// f(D constant, F16 constant) for the narrowest kernel that holds the head. (Long bf16 sequences of narrow heads are better
+// off as heads of 64 on that size's kernels, zero columns and copies included: attention.py brings them there.)
 template <typename F>
 int by_width(int d, int dtype, F f) {
   auto typed = [&](auto width) { return dtype == JG_F16 ? f(width, std::true_type{}) : f(width, std::false_type{}); };

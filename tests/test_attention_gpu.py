@@ -600,3 +600,32 @@ def test_misaligned_heads_of_64_run_the_kernels_that_take_any_alignment(sk, dev)
     acc = torch.zeros(h, sq, d, device=dev)
     rc = lib.jg_attn_fwd(None, None, p(q), p(k), p(v), h, sq, sk, d, scale, None, 0, p(acc), p(lse), bf16, stream)
     assert rc == -2
+
+
+@pytest.mark.parametrize("h,sq,sk,P,d", [(2, 2048, 2048, 2, 40), (1, 2050, 4097, 1, 16), (1, 2048, 1400, 3, 56), (8, 4096, 4096, 1, 32), (2, 2048, 4096, 1, 36)], ids=str)
+def test_narrow_heads_on_long_sequences_run_as_64_columns(h, sq, sk, P, d, dev):
+    """bf16 heads of fewer than 64 columns where the 64-column kernels with zero columns are the faster ones: the ring, the
+    core and the step that merges, against 64 bits; results keep their own width."""
+    torch.manual_seed(sk + d)
+    mk = lambda n: (torch.randn(1, h, n, d, device=dev)).bfloat16()  # noqa: E731
+    q, dout, ks, vs, scale = mk(sq), mk(sq), [mk(sk) for _ in range(P)], [mk(sk) for _ in range(P)], d**-0.5
+    assert ja._as_64_columns(q, ks[0], P) and not ja._as_64_columns(q.half(), ks[0], P) and not ja._as_64_columns(q[..., :1024, :], ks[0], P)
+    leaves = [t.double().requires_grad_() for t in (q, torch.cat(ks, -2), torch.cat(vs, -2))]
+    scores = leaves[0] @ leaves[1].transpose(-1, -2) * scale
+    want_l = torch.logsumexp(scores, -1)
+    want_o = torch.exp(scores - want_l[..., None]) @ leaves[2]
+    want = torch.autograd.grad(want_o, leaves, dout.double())
+    out, lse = ja.ring_forward(q, ks, vs, scale)
+    assert out.shape == q.shape and out.is_contiguous() and rel_l2(out, want_o) < 1e-2 and rel_l2(lse, want_l) < 1e-3
+    dq, dks, dvs = ja.ring_backward(dout, q, out, lse, ks, vs, scale)
+    assert all(t.shape == ks[0].shape and t.is_contiguous() for t in (*dks, *dvs)) and dq.shape == q.shape
+    for got, w in zip((dq, torch.cat(dks, -2), torch.cat(dvs, -2)), want):
+        assert rel_l2(got, w) < 2e-2
+    acc, l_acc = torch.zeros(q.shape, device=dev), torch.full(q.shape[:-1], float("-inf"), device=dev)
+    for k, v in zip(ks, vs):
+        acc, l_acc = ja.attend_step_(q, k, v, scale, acc, l_acc)
+    assert rel_l2(acc, want_o) < 1e-2 and rel_l2(l_acc, want_l) < 1e-3
+    if P == 1:
+        got = ja.core_backward(dout, q, ks[0], vs[0], out, lse, scale)
+        for g, w in zip(got, want):
+            assert g.shape == w.shape and rel_l2(g, w) < 2e-2
