@@ -83,7 +83,7 @@ PRIM_CASES = [
     (2, 8, 5, (12, 40), (3, 1), (1, 1), (1, 0), (1, 1)),
     (1, 16, 16, (5, 10, 34), (1, 1, 1), (1, 1, 1), (0, 0, 0), (1, 1, 1)),
     (1, 8, 8, (6, 9, 20), (3, 1, 3), (1, 1, 1), (1, 0, 0), (1, 1, 1)),
-    # strided 3 x 3 (down-sampling): the stride-1 kernels, sampled / zero-stuffed
+    # strided 3 x 3 (down-sampling): kernels of their own at 2 x 2, else the stride-1 kernels, sampled / zero-stuffed
     (2, 16, 32, (33, 40), (3, 3), (2, 2), (1, 1), (1, 1)),
     (1, 8, 8, (20, 31), (3, 3), (2, 3), (0, 1), (1, 1)),
     (1, 8, 16, (7, 12, 18), (3, 3, 3), (2, 2, 2), (1, 1, 1), (1, 1, 1)),
@@ -216,6 +216,54 @@ def test_odd_rows_and_blocks_of_channels(case, dtype, offset, dev):
     assert rel_l2(gb, g.double().sum(dim=(0, *range(2, 2 + ns)))) < TOL[dtype]
 
 
+# 3 x 3 at stride 2: forward tiles of 64 and of 32 produced channels, one and several of them and of contraction steps; weight
+# gradient blocks of 64 x 64, 64 x 32, 32 x 64 and 32 x 32 channels, several a side, short last ones; rows of several tiles (32
+# produced pixels forward, 64 in the weight gradient) that end inside one; paddings 0 to 2; images whose last row or column
+# no window reaches; many stages a workgroup
+STRIDED_CASES = [
+    (2, 64, 64, (33, 150), (1, 1)),
+    (1, 64, 128, (18, 260), (1, 1)),
+    (2, 32, 64, (20, 71), (2, 2)),
+    (1, 64, 32, (37, 134), (0, 0)),
+    (1, 96, 160, (17, 66), (1, 2)),
+    (2, 128, 64, (9, 259), (2, 0)),
+    (1, 40, 72, (31, 145), (1, 1)),
+    (1, 16, 256, (3, 2), (1, 1)),
+    (4, 64, 64, (130, 514), (1, 1)),
+]
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", STRIDED_CASES, ids=lambda c: f"{c[1]}to{c[2]}_{'x'.join(map(str, c[3]))}_p{c[4][0]}{c[4][1]}")
+def test_strided_3x3_layers_exactly(case, dtype, offset, dev):
+    """Small whole numbers: every product and fp32 sum is exact in any order, so that each cell of the four results is the
+    rounded exact value. ``offset``: elements into its storage at which a tensor starts."""
+    N, ci, co, size, pad = case
+    torch.manual_seed(ci + co)
+
+    def placed(t):
+        flat = torch.empty(t.numel() + offset, dtype=dtype, device=dev)
+        flat[offset:] = t.to(dev, dtype).flatten()
+        return flat[offset:].view(t.shape)
+
+    x = torch.randint(-2, 3, (N, ci, *size)).double()
+    w = torch.randint(-1, 2, (co, ci, 3, 3)).double()
+    b = torch.randint(-3, 4, (co,)).double()
+    args = ((2, 2), pad, (1, 1))
+    y = oc.forward(x, w, b, *args)
+    g = torch.randint(-1, 2, y.shape).double()
+    xg, wg, bg, gg = placed(x), placed(w), placed(b), placed(g)
+    kw = dict(stride=2, padding=pad)
+    same = lambda got, want: got.dtype == dtype and torch.equal(got.cpu(), want.to(dtype))  # noqa: E731
+    assert same(jc.conv_nd(xg, wg, bg, **kw), y)
+    assert same(jc.conv_nd(xg, wg, None, **kw), y - b.view(1, -1, 1, 1))
+    assert same(jc.conv_nd_input(x.shape, wg, gg, **kw), oc.dgrad(x.shape, w, g, *args))
+    gw, gb = jc.conv_nd_weight(xg, w.shape, gg, with_bias_grad=True, **kw)
+    assert same(gw, oc.wgrad(x, w.shape, g, *args)) and same(gb, g.sum(dim=(0, 2, 3)))
+    assert same(jc.conv_nd_weight(xg, w.shape, gg, **kw), oc.wgrad(x, w.shape, g, *args))
+
+
 def test_partial_channel_step_ignores_what_lies_behind_the_last_channel(dev):
     """3 input channels fill 3 of the 16 slots of an MFMA step; the slots behind them are read
     from whatever follows in memory (the next batch entry) and must not reach the result:
@@ -304,6 +352,7 @@ DIST_CASES = [
     ((3, 2), (8, 10), 1, 3, 5, (3, 3), (2, 2), torch.float32, (1, 1), (2, 2)),
     ((2, 2), (16, 32), 1, 32, 32, (3, 3), (1, 2), torch.bfloat16, (2, 1), (1, 2)),
     ((2, 1, 2), (4, 6, 8), 1, 2, 3, (3, 3, 3), (1, 1, 2), torch.float32, (2, 1, 1), (1, 1, 2)),
+    ((2, 2), (32, 160), 2, 64, 128, (3, 3), (1, 1), torch.bfloat16, (2, 2), (1, 1)),
     # need spans that drift against the tiles (halo.py:49-63 with out_local * stride != n): the widths change from rank to rank
     ((2, 2), (16, 20), 2, 4, 6, (3, 3), (0, 0), torch.float32),                    # no padding: (0, 1) and (1, 0)
     ((4, 2), (6, 12), 1, 3, 5, (5, 3), (0, 1), torch.float32),                     # four ranks: (r, 3 - r)
