@@ -134,10 +134,12 @@ def _as_64_columns(q, k, chunks: int = 1) -> bool:
     70/173 and 87/182, 80/204 and 91/196, and 128 heads x 1024 x 2 chunks of 1024 keys 123/329 and 149/374. A width of 32 is a
     kernel's own, and worth leaving only where its four wavefronts a workgroup leave compute units idle: 8 heads x 4096 x
     4096 keys 93/237 and 68/173, 16 heads 106/260 and 121/288."""
-    d, sq, keys = q.shape[-1], q.shape[-2], k.shape[-2] * chunks
-    if q.dtype != torch.bfloat16 or d >= 64 or sq < 2048 or keys < 4096:
+    *lead, sq, d = q.shape
+    if sq < 2048 or d >= 64 or q.dtype != torch.bfloat16:
         return False
-    rows = math.prod(q.shape[:-1])
+    keys, rows = k.shape[-2] * chunks, math.prod(lead) * sq
+    if keys < 4096:
+        return False
     return rows * keys >= 1 << 27 and sq >= 4096 and rows <= 1 << 15 if 24 < d <= 32 else True
 
 
@@ -349,15 +351,16 @@ def _resident_backward(dout, q, out, lse, k_chunks, v_chunks, scale):
     if _as_64_columns(q, k_chunks[0], len(k_chunks)):
         d, P = q.shape[-1], len(k_chunks)
         kv = _chunks_as_64_columns(t.to(q.dtype) for t in (*k_chunks, *v_chunks))
-        dq, dkv = _backward_over(*(_pad_last(t.to(q.dtype), 64) for t in (dout, q, out)), lse, kv[:P], kv[P:], scale)
-        dkv = dkv[..., :d].contiguous()
-        return dq[..., :d].contiguous(), list(dkv[0].unbind(0)), list(dkv[1].unbind(0))
-    dq, dkv = _backward_over(dout, q, out, lse, k_chunks, v_chunks, scale)
-    return dq, list(dkv[0].unbind(0)), list(dkv[1].unbind(0))
+        padded = [_pad_last(t.to(q.dtype), 64) for t in (dout, q, out)]
+        dq, dkv = _backward_over(*padded, lse, kv[:P], kv[P:], scale)[:2]
+        dk, dv = dkv[..., :d].contiguous().unbind(0)
+        return dq[..., :d].contiguous(), list(dk.unbind(0)), list(dv.unbind(0))
+    dq, _, dks, dvs = _backward_over(dout, q, out, lse, k_chunks, v_chunks, scale)
+    return dq, dks, dvs
 
 
 def _backward_over(dout, q, out, lse, k_chunks, v_chunks, scale):
-    """``(dq, dkv)`` of ``jg_attn_bwd_chunks``; ``dkv[0][j]``, ``dkv[1][j]`` are chunk j's dK and dV (one allocation)."""
+    """``(dq, dkv, dks, dvs)`` of ``jg_attn_bwd_chunks``: ``dks``, ``dvs`` are the chunks' views of the one allocation ``dkv``."""
     dout, out, q = _dense(dout.to(q.dtype)), _dense(out.to(q.dtype)), _dense(q)
     lse = lse.to(torch.float32).contiguous()
     ks, vs = [_dense(t.to(q.dtype)) for t in k_chunks], [_dense(t.to(q.dtype)) for t in v_chunks]
@@ -376,7 +379,7 @@ def _backward_over(dout, q, out, lse, k_chunks, v_chunks, scale):
         _lib.stream_ptr(q.device),
     )
     _lib.check(rc, "jg_attn_bwd_chunks")
-    return dq, dkv
+    return dq, dkv, dks, dvs
 
 
 def backward_chunks(dout, q, out, lse, k_chunks, v_chunks, scale):
