@@ -567,7 +567,8 @@ int jg_bias_grad(void* gb, const void* g, int64_t batch, int64_t channels,
                  void* stream);
 
 /* ------------------------------------------------------------------------- *
- * Attention core of the ring step (MFMA kernels: bf16 at head sizes 64, 96, 128; fp16 at 96, 128)
+ * Attention core of the ring step (MFMA kernels: bf16 and fp16 at head sizes that are multiples of 8 up to
+ * 128, fp32 at 32, 64, 128; any lengths)
  *
  * q (batch, sq, d), k / v (batch, sk, d), dense, `batch` = all leading axes
  * flattened (b*h for the "bhsd" layout of jigsaw's sdpa / math cores). One dtype
@@ -588,13 +589,13 @@ int jg_bias_grad(void* gb, const void* g, int64_t batch, int64_t channels,
  * (batch, sq)) are given, this chunk's result is merged into them in place,
  *   w = sigmoid(lse - lse_acc); out_acc += w*(out - out_acc); lse_acc = logaddexp,
  * which is _online_softmax_merge_ (forward.py:23-61) without the round trip of
- * out_j through HBM; `out` / `lse` may then be NULL (bf16 with d = 64, 96 or 128, fp16
- * with d = 96 or 128, sq and sk multiples of 128; fp32 with d = 32, 64 or 128, no bias,
- * 16-byte aligned tensors, any sq and sk; JG_ERR_UNSUPPORTED otherwise).
- * fp32 without a bias at d = 32, 64 or 128 runs on the fp32 matrix-core instructions
- * (forward and backward), other fp32 calls on one-thread-per-row kernels.
- * d must be one of 8, 16, 32, 64, 96, 128 (JG_ERR_UNSUPPORTED otherwise; zero
- * columns appended to q, k, v leave out's other columns and lse unchanged). */
+ * out_j through HBM; `out` / `lse` may then be NULL (bf16 and fp16 with d a multiple of 8
+ * up to 128, fp32 with d = 32, 64 or 128; no bias, 16-byte aligned tensors, any sq and sk;
+ * JG_ERR_UNSUPPORTED otherwise).
+ * Without a bias and with 16-byte aligned tensors those types and head sizes run on the
+ * matrix cores (forward and backward). Everything else runs on one-thread-per-row kernels,
+ * which take any alignment and d = 8, 16, 32, 64, 96, 128 (JG_ERR_UNSUPPORTED otherwise;
+ * zero columns appended to q, k, v leave out's other columns and lse unchanged). */
 int jg_attn_fwd(void* out, float* lse, const void* q, const void* k, const void* v,
                 int64_t batch, int64_t sq, int64_t sk, int64_t d, float scale,
                 const float* bias, int64_t bias_period, float* out_acc,
@@ -604,7 +605,7 @@ int jg_attn_fwd(void* out, float* lse, const void* q, const void* k, const void*
  * _functional/forward.py:160-199, with every chunk here): out (dtype) and lse (fp32) of the queries over all
  * keys; the running maximum, sum and output stay in registers from the first chunk to the last (the
  * reference rounds each step's output before it merges it). k, v are HOST arrays of n_chunks device pointers,
- * read before the call returns. No bias. Covered as jg_attn_bwd_chunks; JG_ERR_UNSUPPORTED otherwise (call
+ * read before the call returns. No bias. Covered as jg_attn_bwd_chunks, but for the workspace; JG_ERR_UNSUPPORTED otherwise (call
  * jg_attn_fwd per chunk with the merge). */
 int jg_attn_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v,
                        int64_t n_chunks, int64_t batch, int64_t sq, int64_t sk, int64_t d, float scale, int dtype,

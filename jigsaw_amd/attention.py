@@ -383,8 +383,10 @@ def _backward_over(dout, q, out, lse, k_chunks, v_chunks, scale):
 
 
 def backward_chunks(dout, q, out, lse, k_chunks, v_chunks, scale):
-    """``(dq, [dk_j], [dv_j])`` over resident chunks in ONE pass (see :func:`ring_backward`). ``None`` for
-    anything but bf16 at head size 64 with lengths that are multiples of 128 and up to 16 chunks of one shape."""
+    """``(dq, [dk_j], [dv_j])`` over resident chunks in ONE pass, a hook for a caller with a loop of its own to fall back to:
+    ``None`` for anything but bf16 at head size 64 with lengths that are multiples of 128 and up to 16 chunks of one
+    shape, where its results have the bits of that loop's. :func:`ring_backward` and the ring's seat take every
+    type, head size and length the kernels cover."""
     if not 1 <= len(k_chunks) <= _MAX_CHUNKS_PER_CALL or len(v_chunks) != len(k_chunks):
         return None
     if q.dtype != torch.bfloat16 or q.shape[-1] != 64 or q.shape[-2] % 128 or k_chunks[0].shape[-2] % 128:

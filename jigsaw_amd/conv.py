@@ -199,7 +199,7 @@ def _embed_weight(w: torch.Tensor, off) -> torch.Tensor:
 
 
 # --------------------------------------------------------------------------- #
-# Strided kernels with extents 1 or 3 (3 x 3 stride 2 down-sampling, ...): the stride-1 result
+# Strided kernels with extents 1 or 3, but for 3 x 3 at stride 2 x 2, which has kernels of its own: the stride-1 result
 # sampled at the stride (forward), and the stride-1 gradients of the output gradient with zeros
 # between its cells (backward). Costs prod(stride) times the matrix-core work of the strided
 # layer and a copy, and still beats the FMA kernels by an order of magnitude.

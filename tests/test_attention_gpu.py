@@ -33,17 +33,17 @@ CORE_SHAPES = [
     (2, 2, 256, 384, 64),  # MFMA path for bf16
     (1, 1, 40, 40, 128),
     (1, 2, 17, 9, 8),
-    (1, 3, 256, 128, 32),  # head size below 64: bf16 runs the head-size-64 MFMA kernels on zero-padded q, k, v
+    (1, 3, 256, 128, 32),  # head sizes below 64: kernels of 32 and 64 columns
     (2, 2, 128, 256, 16),
-    (1, 2, 200, 300, 32),  # ragged queries and keys below head size 64: padded, spare-column key mask
-    (1, 2, 130, 260, 64),  # ragged at head size 64: MFMA on 256 keys + FMA kernel on 4, merged
+    (1, 2, 200, 300, 32),  # ragged queries and keys below head size 64
+    (1, 2, 130, 260, 64),  # ragged at head size 64: 256 keys in the pipeline, 4 behind it
     (2, 1, 128, 130, 16),
     (1, 1, 70, 1000, 64),
     (1, 2, 128, 256, 128),  # head sizes 96 and 128: their own MFMA kernels for bf16
     (2, 2, 256, 128, 96),
     (1, 1, 384, 640, 128),
-    (1, 2, 200, 300, 80),   # padded to head size 96, spare-column key mask
-    (1, 1, 130, 260, 128),  # ragged at head size 128: MFMA on 256 keys + FMA kernel on 4, merged
+    (1, 2, 200, 300, 80),   # the kernel of 96 columns, 16 of them zero
+    (1, 1, 130, 260, 128),  # ragged at head size 128: 256 keys rounded, 4 not
     (1, 1, 70, 200, 96),
     (1, 2, 256, 128, 72),
 ]
@@ -81,7 +81,7 @@ def test_core_forward_backward_match_oracle(shape, dtype, dev):
         (1, 2, 128, 128, 3, torch.bfloat16),  # head sizes 128 and 96: their own kernels, merge fused as well
         (1, 1, 256, 96, 2, torch.bfloat16),
         (1, 2, 128, 128, 2, torch.float16),   # fp16 on the matrix cores, merge fused
-        (1, 2, 256, 64, 2, torch.float16),    # fp16, head size 64: padded to the 96-wide kernels per step
+        (1, 2, 256, 64, 2, torch.float16),    # fp16, head size 64
     ],
 )
 @pytest.mark.parametrize("rank", [0, 2])
