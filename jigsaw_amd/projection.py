@@ -443,9 +443,9 @@ def heads_projection(out: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor
 
 def heads_projection_add(out, weight, bias, residual) -> torch.Tensor:
     """``residual + heads_projection(out, weight, bias)`` with the sum on the GEMM's way out where that exists
-    (bf16, feature counts that are multiples of 8), else in a step of its own."""
+    (bf16, feature counts that are multiples of 8, fewer than 2^31 values), else in a step of its own."""
     n_out, k = weight.shape
-    if (out.dtype == torch.bfloat16 and residual.dtype == torch.bfloat16 and residual.is_contiguous() and out.numel() > 0
+    if (out.dtype == torch.bfloat16 and residual.dtype == torch.bfloat16 and residual.is_contiguous() and 0 < out.numel() < 1 << 31
             and residual.data_ptr() % 16 == 0 and n_out % 8 == 0 and out.shape[-1] % 8 == 0
             and tuple(residual.shape) == (*out.shape[:-3], out.shape[-2], n_out)):
         return _HeadsProjection.apply(out, weight, bias, residual)
