@@ -547,13 +547,13 @@ def test_short_key_ranges_keep_probabilities_in_fp32(h, sq, sk, d, P, dtype, dev
         assert _differ(got, w) < _STRAYS[dtype]
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("h,sq,sk,d,P", [(3, 130, 300, 64, 1), (3, 256, 1000, 64, 3), (30, 256, 1000, 128, 2), (3, 130, 255, 96, 3)], ids=str)
+@pytest.mark.parametrize("h,sq,sk,d,P,dtype", [
+    (3, 130, 300, 64, 1, torch.bfloat16), (3, 256, 1000, 64, 3, torch.bfloat16), (30, 256, 1000, 128, 2, torch.bfloat16),
+    (3, 130, 255, 96, 3, torch.bfloat16), (30, 256, 1000, 128, 2, torch.float16), (3, 130, 255, 96, 3, torch.float16),
+], ids=str)
 def test_keys_behind_the_last_whole_tile_keep_probabilities_in_fp32(h, sq, sk, d, P, dtype, dev):
     """Forward at a head size that fills a kernel: the keys of a chunk behind its last multiple of 128. The whole tiles
     have probabilities near 0 here, so that the last keys alone make the result."""
-    if dtype == torch.float16 and d == 64:
-        pytest.skip("fp16 heads of 64 columns fill no kernel of their own")
     torch.manual_seed(sk + d)
     mk = lambda n: torch.randn(1, h, n, d, device=dev).to(dtype)  # noqa: E731
     q, k, vs, scale = mk(sq), mk(sk), [mk(sk) for _ in range(P)], d**-0.5
