@@ -10,7 +10,7 @@ from __future__ import annotations
 import ctypes
 import threading
 import warnings
-from ctypes import POINTER, c_char_p, c_double, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
+from ctypes import POINTER, c_char_p, c_double, c_float, c_int, c_int32, c_int64, c_size_t, c_uint, c_void_p
 from pathlib import Path
 
 import torch
@@ -195,6 +195,16 @@ SIGNATURES: dict[str, tuple] = {
         c_int,
         [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_float,
          c_int, c_void_p, c_size_t, c_void_p],
+    ),
+    "jg_gn_forward_polls": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_float,
+         c_int, c_uint, c_void_p, c_size_t, c_void_p],
+    ),
+    "jg_gn_backward_polls": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64,
+         c_int64, c_int, c_int, c_uint, c_void_p, c_size_t, c_void_p],
     ),
     "jg_gn_apply_keep": (
         c_int,

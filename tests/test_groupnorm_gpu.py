@@ -212,3 +212,78 @@ def test_input_changed_in_place_before_the_backward(shape, dtype, sharded, dev):
     for a, r in zip(grads, torch.autograd.grad(want, ref, g.double())):
         assert rel_l2(a, r) < max(TOL[dtype], 2e-5)
     assert rel_l2(x, want) < TOL[dtype]
+
+
+@pytest.mark.parametrize("polls", [0, 1, 256])  # separate launches; nearly every chunk left to the second launch; hardly any
+@pytest.mark.parametrize("shape", [
+    # batch, channels, groups, positions; a block keeps 16384 (backward) or 32768 (forward) 16-bit elements, half as many fp32
+    (2, 6, 3, 1), (2, 6, 2, 7), (1, 8, 2, 4097), (1, 4, 2, 16384), (2, 4, 2, 16385), (1, 2, 1, 32777),
+    (1, 8, 1, 9 * 16384 + 5),                         # more chunks than every block adds up itself
+    (1, 64, 2, 16 * 16384), (1, 33, 1, 16 * 16384),   # the most chunks of a group that wait for each other; more
+    (40, 8, 4, 8 * 16384 - 8),                        # more blocks than fit the chip
+    (1, 64, 8, 1 << 20),                              # tensors that go past the last-level cache
+], ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_chunks_kept_in_registers(shape, dtype, polls, dev):
+    """The launches behind ``group_norm`` at the edges of their chunks, whether the blocks of a group meet or not."""
+    from jigsaw_amd import _lib
+
+    N, C, G, S = shape
+    gen = torch.Generator(device=dev).manual_seed(3)
+    x = (torch.randn(N, C, S, device=dev, generator=gen) * 0.5 + 0.3).to(dtype)
+    g = torch.randn(N, C, S, device=dev, generator=gen).to(dtype)
+    w = (1 + 0.2 * torch.randn(C, device=dev, generator=gen)).to(dtype)
+    b = (0.2 * torch.randn(C, device=dev, generator=gen)).to(dtype)
+    lib, p, code = _lib.load(), _lib.ptr, _lib.dtype_code(dtype)
+    y, kept, gx = (torch.full_like(x, float("nan")) for _ in range(3))
+    stats = torch.full((2, N, G), float("nan"), device=dev)
+    gw, gb = torch.full((2, C), float("nan"), device=dev).unbind(0)
+    nbytes = lib.jg_gn_workspace_bytes(N, C, S)
+    ws = torch.full((nbytes,), 255, dtype=torch.uint8, device=dev)
+    rc = lib.jg_gn_forward_polls(p(y), p(kept), p(stats[0]), p(stats[1]), p(x), p(w), p(b), N, C, S, G, 1e-5, code, polls, p(ws), nbytes,
+                                 _lib.stream_ptr(dev))
+    assert rc == 0
+    rc = lib.jg_gn_backward_polls(p(gx), p(gw), p(gb), p(g), p(x), p(stats[0]), p(stats[1]), p(w), N, C, S, G, code, _lib.dtype_code(gw.dtype),
+                                  polls, p(ws), nbytes, _lib.stream_ptr(dev))
+    assert rc == 0 and torch.equal(kept, x)
+    # in fp64, x_hat rounded as the operator rounds it on the way to y
+    xd, gd = x.double().reshape(N, G, -1), (g.double() * w.double()[:, None]).reshape(N, G, -1)
+    mean = xd.mean(-1, keepdim=True)
+    rstd = ((xd - mean).square().mean(-1, keepdim=True) + 1e-5).rsqrt()
+    xn = (xd - mean) * rstd
+    want_gx = rstd * (gd - gd.mean(-1, keepdim=True) - xn * (gd * xn).mean(-1, keepdim=True))
+    xn = xn.reshape(N, C, S)
+    # a rounding to 16 bits of x_hat and one of y (2^-8 bf16, 2^-11 fp16, halved, of values up to 1.5 of the rms); fp32 sums
+    tol = {torch.bfloat16: 4e-3, torch.float16: 5e-4, torch.float32: 3e-6}[dtype]
+    assert rel_l2(y, xn * w.double()[:, None] + b.double()[:, None]) < tol
+    assert rel_l2(stats[0], mean.squeeze(-1)) < 3e-6 and rel_l2(stats[1], rstd.squeeze(-1)) < 3e-6
+    # gx is a difference of terms of the size of rstd g w, which cancel where a group has few elements (two: all but eps)
+    err, term = (gx.double() - want_gx.reshape(N, C, S)).abs(), (rstd * gd).abs()
+    assert err.norm() < tol * term.norm() and err.max() < 8 * tol * term.max()
+    scale = math.sqrt(N * S)  # what a sum of N S values of both signs is measured against
+    assert (gw - (g.double() * xn).sum((0, 2))).abs().max() < 1e-5 * scale + 1e-6 * math.sqrt(N * S) * scale
+    assert (gb - g.double().sum((0, 2))).abs().max() < 1e-5 * scale + 1e-6 * math.sqrt(N * S) * scale
+
+
+def test_group_norm_in_a_captured_graph(dev):
+    """Replays with other inputs, eager work in between, against the eager result."""
+    torch.manual_seed(8)
+    x, g = (torch.randn(2, 32, 64, 130, device=dev).bfloat16() for _ in range(2))
+    w = (1 + 0.2 * torch.randn(32, device=dev)).bfloat16().requires_grad_()
+    x.requires_grad_()
+    step = lambda: (lambda y: [y, *torch.autograd.grad(y, (x, w), g)])(jgn.group_norm(x, 4, w))  # noqa: E731
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for _ in range(3):
+        with torch.no_grad():
+            x.copy_(torch.randn_like(x))
+        graph.replay()
+        got = [t.clone() for t in out]
+        for a, r in zip(got, step()):
+            assert torch.equal(a, r)
