@@ -990,7 +990,7 @@ def _step(x_shape, dtype, w_shape, stride, padding, dilation, ranks, sizes, grou
         tuple(x_shape), lead + geom.padded, launches[0].shape, tuple(w_shape), dtype.itemsize, _lib.dtype_code(dtype),
         address(geom.c_geom(planes)), address(geom.theirs().c_geom(planes)), geom.same_on_every_rank, address(launches[0].desc),
         [launch.nbytes for launch in launches], rows["assemble"], rows["fold"], sent("pack_fwd"), sent("pack_bwd"),
-        fused_fold and dtype == torch.bfloat16 and groups == 1)
+        fused_fold and groups == 1)
 
 
 def _step_for(config, x_shape, x, w, stride, padding, dilation, ranks, sizes):

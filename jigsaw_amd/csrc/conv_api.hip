@@ -101,10 +101,10 @@ extern "C" int jg_conv_dgrad_fold(void* gx, void* const send[27], const void* w,
                "jg_conv_dgrad_fold: axis %d: lo %d + size %d + hi %d != padded extent %d", a, lo[a], n[a],
                geom->hi[a], g.in[a]);
   }
-  if (dtype != JG_BF16 || !jg::mfma_dgrad_supported(g, dtype))
+  if (!jg::mfma_dgrad_supported(g, dtype))
     JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_dgrad_fold: geometry / dtype only has the unfused path");
   return jg::mfma_dgrad_fold(gx, send, lo, n, w, go, g, workspace, workspace_bytes,
-                             static_cast<hipStream_t>(stream));
+                             static_cast<hipStream_t>(stream), dtype);
 }
 
 extern "C" int jg_conv_wgrad(void* gw, const void* x, const void* go, const jg_conv_desc* desc,

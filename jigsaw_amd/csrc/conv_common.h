@@ -48,7 +48,7 @@ int mfma_dgrad(void* gx, const void* w, const void* go, const ConvGeom& g, void*
 // Input gradient split between the unpadded tile and the neighbours' strips: the produced
 // (padded) tensor has extent g.in; [lo, lo + n) of it is the tile.
 int mfma_dgrad_fold(void* gx, void* const strips[27], const int lo[3], const int n[3], const void* w,
-                    const void* go, const ConvGeom& g, void* ws, size_t ws_bytes, hipStream_t s);
+                    const void* go, const ConvGeom& g, void* ws, size_t ws_bytes, hipStream_t s, int dtype);
 // gb (Cout,) or NULL: the bias gradient from the same pass over go
 // xt / tlo / tn: framed input as for mfma_fwd_framed, or NULL
 int mfma_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom& g, void* ws,

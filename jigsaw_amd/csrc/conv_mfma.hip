@@ -344,9 +344,14 @@ __device__ __forceinline__ int px_of_row(int m) { return (m & 0x13) | ((m & 4) <
 // backward for 64 -> 128 channels of 4 x 257 x 257.)
 enum Mode { PLAIN = 0, STRIDED = 1, STRIDED_DGRAD = 2 };
 
-template <int MT, bool EVEN, bool FOLD, bool FRAMED, bool F16 = false, bool PX = false, int MODE = PLAIN>  // MT = produced channels per workgroup: 32 or 64
+// FOLD: the input gradient goes to its owners (see FwdParams::fold). FOLD_WHOLE: bf16, whole tiles of produced channels,
+// stride 1; FOLD_ANY: any type, any number of channels, also the strided gradient.
+enum Fold { FOLD_NONE = 0, FOLD_WHOLE = 1, FOLD_ANY = 2 };
+
+template <int MT, bool EVEN, int FOLD, bool FRAMED, bool F16 = false, bool PX = false, int MODE = PLAIN>  // MT = produced channels per workgroup: 32 or 64
 __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips, FwdParams p) {
-  static_assert(MODE == PLAIN || (!FOLD && !FRAMED), "strided layers have neither the fold epilogue nor the framed input");
+  static_assert(MODE == PLAIN || (FOLD != FOLD_WHOLE && !FRAMED), "strided layers have neither that fold epilogue nor the framed input");
+  static_assert(MODE != STRIDED || !FOLD, "the forward pass has nothing to fold");
   static_assert(MODE != STRIDED_DGRAD || (MT == 32 && !PX), "32 channels of two phases");
   constexpr int ST = MODE == STRIDED ? 2 : 1;
   constexpr int TH = TILE_H / ST, TW = TILE_W / ST;
@@ -897,6 +902,31 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     }
   };
 
+  // store(cb, i, vo) for every channel of the lane that exists, `vo` the byte offset of the channel: it starts at the
+  // lane's first channel and walks by additions (a product per store costs a multiply, a 64-bit add and, with the scalar
+  // registers this kernel has left, a spill reload). Groups of eight channels that do not exist are left out.
+  const int m_here = p.M - mt * MT - ch0;  // channels from the wavefront's first one to the end
+  auto walk_channels = [&](int blocks, uint32_t vo, uint32_t st, auto store) __attribute__((always_inline)) {
+    const uint32_t st8 = 8u * st;
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+      if (cb >= blocks) break;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int have = m_here - cb * 32 - 8 * j;
+        uint32_t v = vo;
+        if (have > 0) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            if (4 * kg + k < have) store(cb, 4 * j + k, v);
+            v += st;
+          }
+        }
+        vo += st8;
+      }
+    }
+  };
+
   auto epilogue_rows = [&](const TileCoord& tc, auto ragged, int free_buf) {
     constexpr bool RAGGED = decltype(ragged)::value;
     const int tw0 = tc.tw * TW + p.org_w;  // first produced column of the tile
@@ -1139,6 +1169,98 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     }
   };
 
+  // The same for any type and number of channels, and for the strided gradient (a lane's two phases are the pixels ow and
+  // ow + 1). One store a pixel (two neighbours of the strided gradient together) and channel, as the epilogues for such
+  // rows have it; bound by the latency of a workgroup's few stages and these stores. It takes 8 to 18 us more than the plain
+  // epilogue at the sizes below, and saves writing the padded gradient, its pack and its fold: gradient to finished fold of
+  // 2 x 72 -> 40 channels of 217 x 301 bf16 56 -> 53 us, of 4 x 128 -> 64 of 256 x 256 at stride 2 72 -> 67 us, of
+  // 4 x 16 -> 3 of 256 x 256 fp32 47 -> 43 us, each with one launch less.
+  auto epilogue_fold_any = [&](const TileCoord& tc) {
+    // The parameters as they are in the kernel-argument segment, read here: held in scalar registers from the kernel's
+    // start on they push the stage loop's own out of them.
+    typedef const __attribute__((address_space(4))) FwdParams* Args;
+    Args args = nullptr;
+#if defined(__HIP_DEVICE_COMPILE__)
+    args = reinterpret_cast<Args>(reinterpret_cast<uintptr_t>((void*)__builtin_amdgcn_kernarg_segment_ptr()) + sizeof(StripTable));
+    asm volatile("" : "+s"(args));
+#endif
+    const __attribute__((address_space(4))) FwdParams& p = *args;
+    constexpr bool PHASES = MODE == STRIDED_DGRAD;
+    const int pa = PHASES ? blockIdx.y & 1 : 0;
+    const int Hp = PHASES ? p.Hx : p.Hout, Wp = PHASES ? p.Wx : p.Wout;  // the produced tensor
+    const int ow = PHASES ? 2 * (tc.tw * TW + wcol0 + ln) - p.px_w : tc.tw * TW + p.org_w + wcol0 + ln;
+    const int od = tc.od;
+    const int rd = od < p.lo_d ? 0 : (od < p.lo_d + p.nD ? 1 : 2);
+    const int cd = od - (rd == 0 ? 0 : (rd == 1 ? p.lo_d : p.lo_d + p.nD));
+    const int ed = rd == 0 ? p.lo_d : (rd == 1 ? p.nD : p.Dout - p.lo_d - p.nD);
+    const size_t plane0 = (size_t)tc.n * p.M + (size_t)mt * MT;
+    const uint32_t es = p.out_kind == 1 ? 4u : 2u;
+    auto region = [](int at, int lo, int n) { return at < lo ? 0 : (at < lo + n ? 1 : 2); };
+    const int hi_h = Hp - p.lo_h - p.nH, hi_w = Wp - p.lo_w - p.nW;
+    const int rw0 = region(ow, p.lo_w, p.nW), rw1 = region(ow + 1, p.lo_w, p.nW);
+    const bool in0 = ow >= 0 && ow < Wp, in1 = PHASES && ow + 1 >= 0 && ow + 1 < Wp;
+    // Values pass through `0 + v`, as in epilogue_fold: the sign of a zero, and of what rounds to one, is cleared
+    auto pair16 = [&](float lo, float hi) {
+      f32x2 v2 = {lo, hi};
+      const uint32_t h2 = F16 ? __builtin_bit_cast(uint32_t, __builtin_convertvector(v2, f16x2)) : __builtin_bit_cast(uint32_t, __builtin_convertvector(v2, bf16x2));
+      uint32_t some;  // a one in every half that is not a zero
+      asm("v_pk_min_u16 %0, %1, %2" : "=v"(some) : "v"(h2 & 0x7fff7fffu), "v"(0x00010001u));
+      return h2 & (some << 15 | 0x7fff7fffu);
+    };
+    const int blocks = PHASES ? 1 : CB;
+#pragma unroll
+    for (int r = 0; r < WROWS; ++r) {
+      const int oh = __builtin_amdgcn_readfirstlane(PHASES ? 2 * (tc.th * TH + wrow0 + r) + pa - p.px_h : tc.th * TH + wrow0 + r);
+      if (oh < 0 || oh >= Hp) continue;
+      const int rh = region(oh, p.lo_h, p.nH);
+      const int ch = oh - (rh == 0 ? 0 : (rh == 1 ? p.lo_h : p.lo_h + p.nH));
+      const int eh = rh == 0 ? p.lo_h : (rh == 1 ? p.nH : hi_h);
+      // (the table's entries by wave-uniform indices: see epilogue_fold)
+      const int slot0 = __builtin_amdgcn_readfirstlane(rd * 9 + rh * 3);
+      // The row's pixels between the edges: a wave-uniform base and a 32-bit lane offset that walks the channels
+      char* const mid = slot0 + 1 == 13 ? reinterpret_cast<char*>(p.y) : static_cast<char*>(strip_entry(slot0 + 1));
+      const uint32_t ps = (uint32_t)ed * (uint32_t)eh * (uint32_t)p.nW, st = es * ps;
+      if (mid != nullptr) {
+        char* const base = mid + es * (plane0 * (size_t)ps + (size_t)((cd * eh + ch) * p.nW));
+        const uint32_t first = 4 * kg * st + es * (uint32_t)(ow - p.lo_w);
+        const bool m0 = in0 && rw0 == 1, m1 = in1 && rw1 == 1;
+        if (p.out_kind == 1) {
+          if (m0) walk_channels(blocks, first, st, [&](int cb, int i, uint32_t vo) { store_f32(base, vo, acc[cb][r][i] + 0.0f); });
+          if (m1) walk_channels(blocks, first + 4, st, [&](int, int i, uint32_t vo) { store_f32(base, vo, acc[CB - 1][r][i] + 0.0f); });
+        } else if (!PHASES) {
+          if (m0)
+            walk_channels(blocks, first, st, [&](int cb, int i, uint32_t vo) {
+              const uint32_t h2 = pair16(acc[cb][r][i & ~1], acc[cb][r][i | 1]);
+              if (i & 1) store_bf16_hi(base, vo, h2);
+              else store_bf16_lo(base, vo, h2);
+            });
+        } else {
+          auto both = [&](int i) { return pair16(acc[0][r][i], acc[CB - 1][r][i]); };
+          if (m0 && m1) walk_channels(blocks, first, st, [&](int, int i, uint32_t vo) { store_4_bytes(base, vo, both(i)); });
+          if (m0 != m1)
+            walk_channels(blocks, m0 ? first : first + 2, st, [&](int, int i, uint32_t vo) { store_bf16_lo(base, vo, m0 ? both(i) : both(i) >> 16); });
+        }
+      }
+      // The few pixels at the edges, each lane with an address of its own
+      auto edge = [&](bool mine, int at, int rw, auto value) __attribute__((always_inline)) {
+        if (__builtin_amdgcn_ballot_w64(mine) == 0) return;
+        char* const lo = static_cast<char*>(strip_entry(slot0));
+        char* const hi = static_cast<char*>(strip_entry(slot0 + 2));
+        char* const to = rw == 0 ? lo : hi;
+        if (!mine || to == nullptr) return;
+        const uint32_t ew = (uint32_t)(rw == 0 ? p.lo_w : hi_w), pe = (uint32_t)ed * (uint32_t)eh * ew;
+        const int cw = rw == 0 ? at : at - p.lo_w - p.nW;
+        const uintptr_t d = reinterpret_cast<uintptr_t>(to) + es * ((plane0 + 4 * kg) * (size_t)pe + (size_t)(cd * eh + ch) * ew + cw);
+        walk_channels(blocks, 0u, es * pe, [&](int cb, int i, uint32_t vo) {
+          if (p.out_kind == 1) *reinterpret_cast<__attribute__((address_space(1))) float*>(d + vo) = value(cb, i) + 0.0f;
+          else *reinterpret_cast<__attribute__((address_space(1))) uint16_t*>(d + vo) = (uint16_t)pair16(value(cb, i), 0.0f);
+        });
+      };
+      edge(in0 && rw0 != 1, ow, rw0, [&](int cb, int i) { return acc[cb][r][i]; });
+      if (PHASES) edge(in1 && rw1 != 1, ow + 1, rw1, [&](int, int i) { return acc[CB - 1][r][i]; });
+    }
+  };
+
   // ---- main loop over the stages (tile, 16-channel step) of this workgroup. The
   // global loads of a stage are issued a whole stage ahead: right after the previous
   // stage's registers were written to LDS, in the middle of the stage before.
@@ -1158,7 +1280,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   // through LDS to leave as 16-byte pieces), and the fold's does where the tile grid lies on the 16-byte grid
   // of the unpadded gradient (the same test as in epilogue_fold; it is the same for every tile of a launch).
   const bool epilogue_uses_lds =
-      MODE == STRIDED_DGRAD ? false : !FOLD || ((((p.org_w - p.lo_w) & 7) == 0) && (p.nW & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
+      MODE == STRIDED_DGRAD || FOLD == FOLD_ANY ? false : !FOLD || ((((p.org_w - p.lo_w) & 7) == 0) && (p.nW & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
   int buf = 0;
   cursor_enter(0);
   issue_stage();
@@ -1224,7 +1346,8 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     // free until the next stage is stored into it. That store waits (barrier above, in the first
     // stage of the next tile) until every wavefront has left this epilogue; until then a
     // wavefront that is done early already runs the next tile's MFMAs.
-    if (FOLD) epilogue_fold(tcur, buf ^ 1);
+    if constexpr (FOLD == FOLD_ANY) epilogue_fold_any(tcur);
+    else if constexpr (FOLD == FOLD_WHOLE) epilogue_fold(tcur, buf ^ 1);
     else epilogue(tcur, buf ^ 1);
   }
 }
@@ -1436,9 +1559,18 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
   int wgs = workgroups_for(tiles, lay.mtiles);
   dim3 grid((unsigned)wgs, (unsigned)lay.mtiles, 1);
   void (*kern)(StripTable, FwdParams) = nullptr;
-  if (L.f16 && (L.fold || L.xt != nullptr))
-    JG_FAIL(JG_ERR_UNSUPPORTED, "%s: the fold epilogue and the framed input are built for bf16 only", who);
-  if (L.mode != PLAIN) {
+  if (L.f16 && L.xt != nullptr)
+    JG_FAIL(JG_ERR_UNSUPPORTED, "%s: the framed input is built for bf16 only", who);
+  if (L.fold && (L.split || L.f16 || phases || lay.mtiles * MT != L.M)) {
+    auto any = [&](auto f16) {
+      constexpr bool F = decltype(f16)::value;
+      if (phases) kern = even ? &conv3x3_mfma_kernel<32, true, FOLD_ANY, false, F, false, STRIDED_DGRAD> : &conv3x3_mfma_kernel<32, false, FOLD_ANY, false, F, false, STRIDED_DGRAD>;
+      else if (MT == 64) kern = even ? &conv3x3_mfma_kernel<64, true, FOLD_ANY, false, F> : &conv3x3_mfma_kernel<64, false, FOLD_ANY, false, F>;
+      else kern = even ? &conv3x3_mfma_kernel<32, true, FOLD_ANY, false, F> : &conv3x3_mfma_kernel<32, false, FOLD_ANY, false, F>;
+    };
+    if (L.f16) any(std::true_type{});
+    else any(std::false_type{});
+  } else if (L.mode != PLAIN) {
     const bool wide = wide_rows && (reinterpret_cast<uintptr_t>(L.y) & 15) == 0;
     auto strided = [&](auto f16, auto px) {
       constexpr bool F = decltype(f16)::value, X = decltype(px)::value;
@@ -1456,8 +1588,8 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
       else strided(std::false_type{}, std::false_type{});
     }
   } else if (L.fold) {
-    if (MT == 64) kern = even ? &conv3x3_mfma_kernel<64, true, true, false> : &conv3x3_mfma_kernel<64, false, true, false>;
-    else kern = even ? &conv3x3_mfma_kernel<32, true, true, false> : &conv3x3_mfma_kernel<32, false, true, false>;
+    if (MT == 64) kern = even ? &conv3x3_mfma_kernel<64, true, FOLD_WHOLE, false> : &conv3x3_mfma_kernel<64, false, FOLD_WHOLE, false>;
+    else kern = even ? &conv3x3_mfma_kernel<32, true, FOLD_WHOLE, false> : &conv3x3_mfma_kernel<32, false, FOLD_WHOLE, false>;
   } else if (L.xt != nullptr) {
     if (MT == 64) kern = even ? &conv3x3_mfma_kernel<64, true, false, true> : &conv3x3_mfma_kernel<64, false, false, true>;
     else kern = even ? &conv3x3_mfma_kernel<32, true, false, true> : &conv3x3_mfma_kernel<32, false, false, true>;
@@ -1638,16 +1770,12 @@ int mfma_dgrad(void* gx, const void* w, const void* go, const ConvGeom& g, void*
 }
 
 int mfma_dgrad_fold(void* gx, void* const strips[27], const int lo[3], const int n[3], const void* w,
-                    const void* go, const ConvGeom& g, void* ws, size_t ws_bytes, hipStream_t s) {
-  if (g.s[2] != 1) JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_dgrad_fold(mfma): strided layers only have the unfused path");
-  // the fold epilogue has no path for a ragged last tile of produced channels
-  const Layout lay = layout_of(g.k[0] * pad16(g.cout), g.cin);
-  if (lay.mtiles * lay.MT != g.cin)
-    JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_dgrad_fold(mfma): %d input channels are not a multiple of %d", g.cin, lay.MT);
-  // the epilogue addresses the MT channel planes of a tile through a 32-bit byte offset
-  if ((long long)n[0] * n[1] * n[2] * 2 * lay.MT >= (1ll << 32) || (long long)g.in[0] * g.in[1] * g.in[2] * 2 * lay.MT >= (1ll << 32))
-    JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_dgrad_fold(mfma): %d planes of the tile do not fit a 32-bit offset", lay.MT);
-  return dgrad_launch(gx, strips, lo, n, w, go, g, ws, ws_bytes, s, "jg_conv_dgrad_fold(mfma)");
+                    const void* go, const ConvGeom& g, void* ws, size_t ws_bytes, hipStream_t s, int dtype) {
+  // the epilogues address the MT channel planes of a tile through a 32-bit byte offset
+  const int MT = layout_of(g.k[0] * pad16(g.cout), g.cin, g.s[2] == 2).MT, es = dtype == JG_F32 ? 4 : 2;
+  if ((long long)n[0] * n[1] * n[2] * es * MT >= (1ll << 32) || (long long)g.in[0] * g.in[1] * g.in[2] * es * MT >= (1ll << 32))
+    JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_dgrad_fold(mfma): %d planes of the tile do not fit a 32-bit offset", MT);
+  return dgrad_launch(gx, strips, lo, n, w, go, g, ws, ws_bytes, s, "jg_conv_dgrad_fold(mfma)", dtype);
 }
 
 }  // namespace jg

@@ -11,6 +11,7 @@ import pytest
 import torch
 
 from helpers import conv_geometry, mesh_coords, neighbour, rel_l2
+from jigsaw_amd import _lib
 from jigsaw_amd import conv as jc
 from jigsaw_amd.halo import halo_pack
 from oracle import conv as oc
@@ -771,3 +772,48 @@ def test_config3_full_size_properties(dev):
     want0 = oc.wgrad(x_aug[0:1].float().cpu(), w.shape, g[0:1].float().cpu(), (1, 1, 1), (0, 0, 0), (1, 1, 1))
     assert rel_l2(parts[0], want0) < 2e-2
     assert rel_l2(gb, g.float().sum((0, 2, 3, 4))) < 1e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("case", [
+    # size, lo, hi, conv padding on the padded tile, stride, N, c_in, c_out, strips present
+    ((17, 23), (1, 1), (1, 1), (0, 0), 1, 2, 40, 24, "all"),       # ragged channels, odd rows
+    ((33, 65), (1, 1), (1, 1), (0, 0), 1, 1, 3, 16, "all"),
+    ((16, 62), (0, 1), (1, 0), (1, 0), 1, 1, 72, 8, "some"),       # the padded row is a tile; one axis padded by the conv
+    ((16, 130), (2, 1), (0, 1), (0, 0), 1, 1, 65, 16, "all"),
+    ((5, 9, 33), (1, 1, 1), (1, 1, 1), (0, 0, 0), 1, 1, 5, 7, "some"),
+    ((16, 32), (1, 1), (0, 0), (0, 0), 2, 2, 32, 24, "all"),       # stride 2: whole and ragged channel tiles
+    ((34, 66), (1, 1), (0, 0), (0, 0), 2, 1, 40, 16, "all"),
+    ((34, 66), (0, 0), (0, 0), (1, 1), 2, 1, 7, 16, "all"),
+    ((32, 130), (1, 0), (1, 0), (0, 1), 2, 1, 33, 16, "some"),
+], ids=str)
+def test_fused_dgrad_fold_any_channels_types_and_strides(case, dtype, dev):
+    """jg_conv_dgrad_fold == jg_conv_dgrad and halo_pack, bit for bit, the sign of zeros cleared."""
+    from jigsaw_amd.halo import HaloGeometry, halo_fold, new_strips
+
+    size, lo, hi, pad, stride, N, ci, co, which = case
+    ns = len(size)
+    geom = HaloGeometry(size, lo, hi)
+    torch.manual_seed(4)
+    out_sp = tuple((geom.padded[a] + 2 * pad[a] - 3) // stride + 1 for a in range(ns))
+    w = ((torch.rand(co, ci, *(3,) * ns, device=dev) * 2 - 1) / (co * 3**ns) ** 0.5).to(dtype)
+    g = torch.randn(N, co, *out_sp, device=dev).to(dtype)
+    g[0].mul_(1e-7 if dtype == torch.float16 else 1e-38)  # results that round to zero, of both signs
+    offs = [o for o in geom.offsets() if all(geom.strip_extent(o, "pack_bwd")[a] > 0 for a in range(ns))]
+    if which == "some":
+        offs = offs[::2]
+    want = jc.conv_nd_input((N, ci, *geom.padded), w, g, stride=stride, padding=pad)
+    want_send = halo_pack(want, geom, from_padded=True, present=offs) if offs else {}
+    launch = jc._launch_for(1, dtype, (N, ci, *geom.padded), w.shape, (stride,) * ns, pad, (1,) * ns, 1)
+    send, tab = new_strips(geom, "pack_bwd", (N, ci), tuple(offs), dtype, dev)
+    for t in send.values():
+        t.fill_(7)
+    gx = torch.full((N, ci, *size), 7.0, dtype=dtype, device=dev)
+    ws = jc._scratch(launch, dev)
+    rc = _lib.load().jg_conv_dgrad_fold(_lib.ptr(gx), tab, _lib.ptr(w), _lib.ptr(g), launch.desc, geom.c_geom(N * ci), _lib.dtype_code(dtype),
+                                        _lib.ptr(ws), launch.nbytes, _lib.stream_ptr(dev))
+    assert rc == 0, _lib.load().jg_last_error()
+    bits = {torch.float32: torch.int32}.get(dtype, torch.int16)
+    assert torch.equal(gx.view(bits), halo_fold(want, {}, geom).view(bits))
+    for o in offs:
+        assert torch.equal(send[o].view(bits), (want_send[o] + 0).view(bits)), f"strip {o}"
