@@ -289,7 +289,8 @@ def ring_forward(q, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.T
     rounded before it is merged, as it is step by step)."""
     P = len(k_chunks)
     order = [(rank + step) % P for step in range(P)]
-    one_pass = _resident_forward(q, [k_chunks[j] for j in order], [v_chunks[j] for j in order], scale)
+    ks, vs = [k_chunks[j] for j in order], [v_chunks[j] for j in order]
+    one_pass = _native("ring_forward", q, ks, vs, scale) or _resident_forward(q, ks, vs, scale)
     if one_pass is not None:
         return one_pass
     acc = torch.promote_types(q.dtype, torch.float32)
@@ -318,6 +319,13 @@ def _pointers(tensors) -> ctypes.Array:
 def _chunks_as_64_columns(chunks) -> list:
     """The chunks with zero columns up to 64: three launches for all of them."""
     return list(_pad_last(torch.stack(tuple(chunks)), 64).unbind(0))
+
+
+def _native(name, *args):
+    """The native host module's version of a resident call (``csrc/host.cpp``): 16-bit chunks on the GPU that need no copy,
+    conversion or zero columns. ``None`` for all others, and without the module."""
+    host = _lib.host() if args[0].is_cuda else None
+    return None if host is None else getattr(host, name)(*args, _lib.stream_handle(args[0].device))
 
 
 def _resident_forward(q, k_chunks, v_chunks, scale):
@@ -404,7 +412,8 @@ def ring_backward(dout, q, out, lse, k_chunks, v_chunks, scale):
     dK/dV over the ranks that attended a chunk is the caller's collective. Chunks that are all
     resident go through one pass (``jg_attn_bwd_chunks``) where it covers them."""
     core = q.dtype
-    one_pass = _resident_backward(dout, q, out, lse, k_chunks, v_chunks, scale)
+    one_pass = (_native("ring_backward", dout, q, out, lse, list(k_chunks), list(v_chunks), scale)
+                or _resident_backward(dout, q, out, lse, k_chunks, v_chunks, scale))
     if one_pass is not None:
         return one_pass
     dout, out = dout.to(core), out.to(core)

@@ -1,4 +1,7 @@
-// Host side of the distributed convolution's step: allocations, strips, pointer tables and the calls into
+// Host side of the small steps in native code: the distributed convolution (Step), ring attention over resident chunks, the
+// sharded LayerNorm's pieces between its collectives, GroupNorm of a whole tensor.
+//
+// The convolution: allocations, strips, pointer tables and the calls into
 // libjigsaw_hip.so, in native code. A step of one layer is 10 launches of 3 to 60 us; worked through Python
 // functions (checks, tuples of shapes, 14 allocations, up to 26 strips cut and looked up, ctypes calls) the host
 // took about 165 us for it beside autograd's own 60, which is what small and ordinary layers then ran at
@@ -238,6 +241,201 @@ class Step {
   std::atomic<bool> fold_;
 };
 
+// ---- attention and norms: checks, allocations and calls of the Python routes in attention.py, layernorm.py, groupnorm.py,
+// for tensors that need no conversion or copy; None for all others, before anything is allocated. Host time of a step, with
+// autograd's own: ring of 4 heads x 128 x 2 chunks 49 us through Python, 20 here;
+// LayerNorm of 4096 x 256 of 512 173 and 136 (its four collectives included); GroupNorm of 2 x 32 x 60 x 70 142 and 111.
+
+int code_of(const at::Tensor& t) {
+  switch (t.scalar_type()) {
+    case at::kFloat: return JG_F32;
+    case at::kBFloat16: return JG_BF16;
+    case at::kHalf: return JG_F16;
+    default: return -1;
+  }
+}
+bool on_gpu(const at::Tensor& t) { return t.is_cuda() && t.is_contiguous(); }
+bool aligned(const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+void* pointer(uintptr_t p) { return reinterpret_cast<void*>(p); }
+
+using List = std::vector<at::Tensor>;
+constexpr size_t kMostChunks = 16;       // attention._MAX_CHUNKS_PER_CALL
+constexpr int64_t kMostBatch = 65535;    // attention._MOST_BATCH
+constexpr int64_t kMostRows = 1 << 23;   // attention._MOST_ROWS
+
+// What the one-pass kernels take without copies, conversions or zero columns (attention._resident, _as_64_columns)
+bool ring_ok(const at::Tensor& q, const List& k, const List& v, int64_t* batch) {
+  const int64_t n = q.dim();
+  if (n < 3 || k.empty() || k.size() > kMostChunks || v.size() != k.size() || q.numel() == 0 || k[0].numel() == 0) return false;
+  const int64_t d = q.size(-1), sq = q.size(-2), sk = k[0].dim() == n ? k[0].size(-2) : 0;
+  if ((q.scalar_type() != at::kBFloat16 && q.scalar_type() != at::kHalf) || d % 8 != 0 || d > 128 || sq > kMostRows || sk > kMostRows) return false;
+  if (q.scalar_type() == at::kBFloat16 && d < 64 && sq >= 2048 && sk * (int64_t)k.size() >= 4096) return false;
+  *batch = q.numel() / (sq * d);
+  if (*batch > kMostBatch || !on_gpu(q) || !aligned(q)) return false;
+  for (int64_t a = 0; a < n; ++a)
+    if (a != n - 2 && (k[0].dim() != n || k[0].size(a) != q.size(a))) return false;
+  for (size_t j = 0; j < k.size(); ++j)
+    for (const at::Tensor* t : {&k[j], &v[j]})
+      if (t->sizes() != k[0].sizes() || t->scalar_type() != q.scalar_type() || t->device() != q.device() || !t->is_contiguous() || !aligned(*t))
+        return false;
+  return true;
+}
+
+template <typename P>
+void addresses(const List& from, P* to) {
+  for (size_t j = 0; j < from.size(); ++j) to[j] = from[j].data_ptr();
+}
+
+py::object ring_forward(const at::Tensor& q, const List& k, const List& v, double scale, uintptr_t stream) {
+  int64_t batch;
+  if (!ring_ok(q, k, v, &batch)) return py::none();
+  at::AutoDispatchBelowADInplaceOrView below;
+  const at::Tensor out = at::empty_like(q), lse = at::empty(q.sizes().slice(0, q.dim() - 1), q.options().dtype(at::kFloat));
+  const void *kp[kMostChunks], *vp[kMostChunks];
+  addresses(k, kp);
+  addresses(v, vp);
+  check(jg_attn_fwd_chunks(out.data_ptr(), lse.data_ptr<float>(), q.data_ptr(), kp, vp, k.size(), batch, q.size(-2), k[0].size(-2),
+                           q.size(-1), (float)scale, code_of(q), pointer(stream)),
+        "jg_attn_fwd_chunks");
+  return py::make_tuple(out, lse);
+}
+
+py::object ring_backward(const at::Tensor& dout, const at::Tensor& q, const at::Tensor& out, const at::Tensor& lse, const List& k,
+                         const List& v, double scale, uintptr_t stream) {
+  int64_t batch;
+  if (!ring_ok(q, k, v, &batch)) return py::none();
+  for (const at::Tensor* t : {&dout, &out})
+    if (t->sizes() != q.sizes() || t->scalar_type() != q.scalar_type() || t->device() != q.device() || !t->is_contiguous() || !aligned(*t)) return py::none();
+  if (lse.scalar_type() != at::kFloat || lse.device() != q.device() || !lse.is_contiguous() || lse.sizes() != q.sizes().slice(0, q.dim() - 1))
+    return py::none();
+  at::AutoDispatchBelowADInplaceOrView below;
+  const int64_t sq = q.size(-2), sk = k[0].size(-2), d = q.size(-1), P = (int64_t)k.size();
+  Shape both{2 * P};
+  both.append(k[0].sizes().begin(), k[0].sizes().end());
+  const at::Tensor dq = at::empty_like(q), dkv = at::empty(both, q.options());
+  const List views = dkv.unbind(0);
+  const List dk(views.begin(), views.begin() + P), dv(views.begin() + P, views.end());
+  const size_t nbytes = jg_attn_bwd_workspace_bytes(batch, sq, sk, d);
+  const at::Tensor ws = at::empty({(int64_t)(nbytes > 4 ? nbytes : 4)}, q.options().dtype(at::kByte));
+  const void *kp[kMostChunks], *vp[kMostChunks];
+  void *dkp[kMostChunks], *dvp[kMostChunks];
+  addresses(k, kp);
+  addresses(v, vp);
+  addresses(dk, dkp);
+  addresses(dv, dvp);
+  check(jg_attn_bwd_chunks(dq.data_ptr(), dkp, dvp, dout.data_ptr(), q.data_ptr(), kp, vp, P, out.data_ptr(), lse.data_ptr<float>(),
+                           batch, sq, sk, d, (float)scale, code_of(q), ws.data_ptr(), nbytes, pointer(stream)),
+        "jg_attn_bwd_chunks");
+  return py::make_tuple(dq, dk, dv);
+}
+
+// (mean, var, the rank's own mean, room for the root): the row statistics before the collectives
+py::object ln_partial(const at::Tensor& x, bool sharded, uintptr_t stream) {
+  if (x.dim() < 1 || x.numel() == 0 || !on_gpu(x) || code_of(x) < 0) return py::none();
+  at::AutoDispatchBelowADInplaceOrView below;
+  const int64_t cols = x.size(-1), rows = x.numel() / cols;
+  Shape shape{4};
+  shape.append(x.sizes().begin(), x.sizes().end() - 1);
+  shape.push_back(1);
+  const List t = at::empty(shape, x.options().dtype(at::kFloat)).unbind(0);
+  check(jg_ln_partial_fwd2(t[0].data_ptr<float>(), sharded ? t[2].data_ptr<float>() : nullptr, t[1].data_ptr<float>(), x.data_ptr(), rows, cols,
+                           code_of(x), pointer(stream)),
+        "jg_ln_partial_fwd2");
+  return py::make_tuple(t[0], t[1], t[2], t[3]);
+}
+
+void ln_recentre(const at::Tensor& var, const at::Tensor& own, const at::Tensor& mean, uintptr_t stream) {
+  check(jg_ln_recentre(var.data_ptr<float>(), own.data_ptr<float>(), mean.data_ptr<float>(), var.numel(), pointer(stream)), "jg_ln_recentre");
+}
+
+// (y, x_norm, var + eps) in w's type; `std` gets the root. x, w and b as the Python route has them at this point.
+py::tuple ln_apply(const at::Tensor& x, const at::Tensor& mean, const at::Tensor& var, const at::Tensor& std, const at::Tensor& w,
+                   const c10::optional<at::Tensor>& b, double eps, uintptr_t stream) {
+  at::AutoDispatchBelowADInplaceOrView below;
+  const int64_t cols = x.size(-1), rows = x.numel() / cols;
+  const at::Tensor y = at::empty(x.sizes(), w.options()), x_norm = at::empty(x.sizes(), w.options()), var_eps = at::empty(mean.sizes(), w.options());
+  check(jg_ln_apply2(y.data_ptr(), x_norm.data_ptr(), std.data_ptr<float>(), var_eps.data_ptr(), x.data_ptr(), mean.data_ptr<float>(),
+                     var.data_ptr<float>(), w.data_ptr(), b ? b->data_ptr() : nullptr, rows, cols, (float)eps, code_of(x), code_of(w), pointer(stream)),
+        "jg_ln_apply2");
+  return py::make_tuple(y, x_norm, var_eps);
+}
+
+// (mean of g w, sum of g w x_norm, gw, gb): the backward before the collectives; parameter gradients in `like`'s type
+py::object ln_partial_bwd(const at::Tensor& g, const at::Tensor& x_norm, const at::Tensor& w, const at::Tensor& std, bool need_w, bool need_b,
+                          const at::ScalarType grad_type, uintptr_t stream) {
+  if (g.numel() == 0 || !on_gpu(g) || !on_gpu(x_norm) || !on_gpu(w) || g.scalar_type() != x_norm.scalar_type() || g.sizes() != x_norm.sizes() ||
+      w.scalar_type() != g.scalar_type() || code_of(g) < 0)
+    return py::none();
+  at::AutoDispatchBelowADInplaceOrView below;
+  const int64_t cols = g.size(-1), rows = g.numel() / cols;
+  Shape shape{2};
+  shape.append(std.sizes().begin(), std.sizes().end());
+  const List t = at::empty(shape, std.options()).unbind(0);
+  const auto options = g.options().dtype(grad_type);
+  const at::Tensor gw = need_w ? at::empty({cols}, options) : at::Tensor(), gb = need_b ? at::empty({cols}, options) : at::Tensor();
+  const size_t nbytes = need_w || need_b ? jg_ln_bwd_workspace_bytes(rows, cols) : 0;
+  const at::Tensor ws = at::empty({(int64_t)(nbytes > 4 ? nbytes : 4)}, g.options().dtype(at::kByte));
+  const int code = grad_type == at::kFloat ? JG_F32 : grad_type == at::kBFloat16 ? JG_BF16 : JG_F16;
+  check(jg_ln_partial_bwd2(t[0].data_ptr<float>(), t[1].data_ptr<float>(), need_w ? gw.data_ptr() : nullptr, need_b ? gb.data_ptr() : nullptr, code,
+                           g.data_ptr(), x_norm.data_ptr(), w.data_ptr(), rows, cols, code_of(g), ws.data_ptr(), nbytes, pointer(stream)),
+        "jg_ln_partial_bwd2");
+  return py::make_tuple(t[0], t[1], need_w ? py::cast(gw) : py::none(), need_b ? py::cast(gb) : py::none());
+}
+
+at::Tensor ln_bwd_apply(const at::Tensor& g, const at::Tensor& x_norm, const at::Tensor& w, const at::Tensor& mean, const at::Tensor& dot,
+                        const at::Tensor& std, int64_t n_global, uintptr_t stream) {
+  at::AutoDispatchBelowADInplaceOrView below;
+  const int64_t cols = g.size(-1), rows = g.numel() / cols;
+  const at::Tensor gx = at::empty_like(g);
+  check(jg_ln_bwd_apply(gx.data_ptr(), g.data_ptr(), x_norm.data_ptr(), w.data_ptr(), mean.data_ptr<float>(), dot.data_ptr<float>(),
+                        std.data_ptr<float>(), rows, cols, n_global, code_of(g), pointer(stream)),
+        "jg_ln_bwd_apply");
+  return gx;
+}
+
+bool like_channels(const c10::optional<at::Tensor>& t, const at::Tensor& x) {
+  return !t || (on_gpu(*t) && t->scalar_type() == x.scalar_type() && t->device() == x.device() && t->dim() == 1 && t->size(0) == x.size(1));
+}
+
+// (y, the copy of x or None, mean, rstd)
+py::object gn_forward(const at::Tensor& x, int64_t groups, const c10::optional<at::Tensor>& w, const c10::optional<at::Tensor>& b, double eps,
+                      bool keep, uintptr_t stream) {
+  if (x.dim() < 2 || x.numel() == 0 || !on_gpu(x) || code_of(x) < 0 || !like_channels(w, x) || !like_channels(b, x)) return py::none();
+  at::AutoDispatchBelowADInplaceOrView below;
+  const int64_t n = x.size(0), c = x.size(1), s = x.numel() / (n * c);
+  const at::Tensor y = at::empty_like(x), kept = keep ? at::empty_like(x) : at::Tensor();
+  const List t = at::empty({2, n, groups}, x.options().dtype(at::kFloat)).unbind(0);
+  const size_t nbytes = jg_gn_workspace_bytes(n, c, s);
+  const at::Tensor ws = at::empty({(int64_t)nbytes}, x.options().dtype(at::kByte));
+  check(jg_gn_forward_keep(y.data_ptr(), keep ? kept.data_ptr() : nullptr, t[0].data_ptr<float>(), t[1].data_ptr<float>(), x.data_ptr(),
+                           w ? w->data_ptr() : nullptr, b ? b->data_ptr() : nullptr, n, c, s, groups, (float)eps, code_of(x), ws.data_ptr(), nbytes,
+                           pointer(stream)),
+        "jg_gn_forward_keep");
+  return py::make_tuple(y, keep ? py::cast(kept) : py::none(), t[0], t[1]);
+}
+
+// (gx, gw, gb); the parameter gradients in `grad_type`
+py::object gn_backward(const at::Tensor& g, const at::Tensor& x, const at::Tensor& mean, const at::Tensor& rstd, const c10::optional<at::Tensor>& w,
+                       int64_t groups, bool need_x, bool need_w, bool need_b, const at::ScalarType grad_type, uintptr_t stream) {
+  if (g.numel() == 0 || !on_gpu(g) || !on_gpu(x) || g.scalar_type() != x.scalar_type() || g.sizes() != x.sizes() || code_of(g) < 0 ||
+      !like_channels(w, x))
+    return py::none();
+  at::AutoDispatchBelowADInplaceOrView below;
+  const int64_t n = x.size(0), c = x.size(1), s = x.numel() / (n * c);
+  const auto options = g.options().dtype(grad_type);
+  const at::Tensor gx = need_x ? at::empty_like(g) : at::Tensor(), gw = need_w ? at::empty({c}, options) : at::Tensor(),
+                   gb = need_b ? at::empty({c}, options) : at::Tensor();
+  const size_t nbytes = jg_gn_workspace_bytes(n, c, s);
+  const at::Tensor ws = at::empty({(int64_t)nbytes}, x.options().dtype(at::kByte));
+  const int code = grad_type == at::kFloat ? JG_F32 : grad_type == at::kBFloat16 ? JG_BF16 : JG_F16;
+  check(jg_gn_backward(need_x ? gx.data_ptr() : nullptr, need_w ? gw.data_ptr() : nullptr, need_b ? gb.data_ptr() : nullptr, g.data_ptr(), x.data_ptr(),
+                       mean.data_ptr<float>(), rstd.data_ptr<float>(), w ? w->data_ptr() : nullptr, n, c, s, groups, code_of(x), code,
+                       ws.data_ptr(), nbytes, pointer(stream)),
+        "jg_gn_backward");
+  auto given = [](const at::Tensor& t) -> py::object { return t.defined() ? py::cast(t) : py::none(); };
+  return py::make_tuple(given(gx), given(gw), given(gb));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -249,4 +447,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       .def("forward", &Step::forward)
       .def("backward", &Step::backward)
       .def("finish", &Step::finish);
+  m.def("ring_forward", &ring_forward);
+  m.def("ring_backward", &ring_backward);
+  m.def("ln_partial", &ln_partial);
+  m.def("ln_recentre", &ln_recentre);
+  m.def("ln_apply", &ln_apply);
+  m.def("ln_partial_bwd", &ln_partial_bwd);
+  m.def("ln_bwd_apply", &ln_bwd_apply);
+  m.def("gn_forward", &gn_forward);
+  m.def("gn_backward", &gn_backward);
 }

@@ -186,9 +186,18 @@ class _GroupNormOutput(torch.autograd.Function):
         cdt = _compute_dtype(x)
         given, x = x, x.to(cdt).contiguous()
         # a cast or a rearrangement is a copy already
-        kept = torch.empty_like(x) if grad and any(ctx.needs_input_grad) and x.data_ptr() == given.data_ptr() else None
+        keep = grad and any(ctx.needs_input_grad) and x.data_ptr() == given.data_ptr()
         w = None if weight is None else weight.to(cdt).contiguous()
         b = None if bias is None else bias.to(cdt).contiguous()
+        ctx.num_groups, ctx.spatial_groups = num_groups, spatial_groups
+        ctx.dtypes = (None if weight is None else weight.dtype, None if bias is None else bias.dtype)
+        host = None if spatial_groups else _lib.host()
+        done = None if host is None else host.gn_forward(x, num_groups, w, b, float(eps), keep, _lib.stream_handle(x.device))
+        if done is not None:  # the same calls as below
+            y, kept, mean, rstd = done
+            ctx.save_for_backward(x if kept is None else kept, mean, rstd, None, w)
+            return y
+        kept = torch.empty_like(x) if keep else None
         n, c, s = _dims(x)
         lib, dev, code = _lib.load(), x.device, _lib.dtype_code(cdt)
         y = torch.empty_like(x)
@@ -205,8 +214,6 @@ class _GroupNormOutput(torch.autograd.Function):
                                         _lib.ptr(b), n, c, s, num_groups, float(eps), code, _lib.ptr(ws), nbytes,
                                         _lib.stream_ptr(dev))
             _lib.check(rc, "jg_gn_forward_keep")
-        ctx.num_groups, ctx.spatial_groups = num_groups, spatial_groups
-        ctx.dtypes = (None if weight is None else weight.dtype, None if bias is None else bias.dtype)
         ctx.save_for_backward(x if kept is None else kept, mean, rstd, count, w)
         return y
 
@@ -225,6 +232,11 @@ class _GroupNormOutput(torch.autograd.Function):
         gdt = next((d for d in (dt_w, dt_b) if d in _lib._DTYPES), torch.float32)
         if dt_w is not None and dt_b is not None and dt_w != dt_b:
             gdt = torch.float32
+        host = None if ctx.spatial_groups else _lib.host()
+        done = None if host is None else host.gn_backward(g, x, mean, rstd, w, groups, need_x, need_w, need_b, gdt, _lib.stream_handle(g.device))
+        if done is not None:  # the same calls as below
+            gx, gw, gb = done
+            return gx, None, None if gw is None else gw.to(dt_w), None if gb is None else gb.to(dt_b), None, None, None
         gw = torch.empty(c, dtype=gdt, device=dev) if need_w else None
         gb = torch.empty(c, dtype=gdt, device=dev) if need_b else None
         gx = torch.empty_like(g) if need_x else None

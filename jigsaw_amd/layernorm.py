@@ -74,11 +74,23 @@ class _LayerNorm(PositionalFunction):
         x = x.contiguous()
         w = weight.to(cdt).contiguous()
         b = None if bias is None else bias.to(cdt).contiguous()
+        sharded, host = _group_size(channel_group) > 1, _lib.host()
+        if host is not None:  # the same calls as below
+            handle = _lib.stream_handle(x.device)
+            stats = host.ln_partial(x, sharded, handle)
+            if stats is not None:
+                mean, var, local_mean, std = stats
+                if sharded:
+                    _all_reduce(mean, "avg", channel_group)
+                    host.ln_recentre(var, local_mean, mean, handle)
+                    _all_reduce(var, "avg", channel_group)
+                y, x_norm, var_eps = host.ln_apply(x, mean, var, std, w, b, float(eps), handle)
+                var_eps._jg_std = std
+                return y, x_norm, (w.view_as(w) if w is weight else w), var_eps
         cols = x.shape[-1]
         rows = x.numel() // cols
         lib, dev, stream = _lib.load(), x.device, _lib.stream_ptr(x.device)
         stat_shape = x.shape[:-1] + (1,)
-        sharded = _group_size(channel_group) > 1
         # the mean that is averaged over the group, the variance, the rank's own mean, and the root the backward wants
         mean, var, local_mean, std = torch.empty((4, *stat_shape), dtype=torch.float32, device=dev).unbind(0)
         rc = lib.jg_ln_partial_fwd2(_lib.ptr(mean), _lib.ptr(local_mean if sharded else None), _lib.ptr(var), _lib.ptr(x),
@@ -126,15 +138,28 @@ class _LayerNorm(PositionalFunction):
         cols = x_norm.shape[-1]
         rows = x_norm.numel() // cols
         n_global = cols * _group_size(group)
-        lib = _lib.load()
         dev = g.device
 
-        mean_gxn, dot = torch.empty((2, *std.shape), dtype=torch.float32, device=dev).unbind(0)
-        need_w = ctx.needs_input_grad[1]
+        need_x, need_w = ctx.needs_input_grad[:2]
         need_b = ctx.has_bias and ctx.needs_input_grad[2]
         # the column sums leave the kernel in the parameters' dtype where they share one
         wdt, bdt = ctx.param_dtypes
         gdt = wdt if wdt in _lib._DTYPES and bdt in (None, wdt) else torch.float32
+        host = _lib.host()
+        if host is not None:  # the same calls as below
+            handle = _lib.stream_handle(dev)
+            parts = host.ln_partial_bwd(g, x_norm, w, std, need_w, need_b, gdt, handle)
+            if parts is not None:
+                mean_gxn, dot, gw, gb = parts
+                grad_x = None
+                if need_x:
+                    _all_reduce(mean_gxn, "avg", group)
+                    _all_reduce(dot, "sum", group)
+                    grad_x = host.ln_bwd_apply(g, x_norm, w, mean_gxn, dot, std, n_global, handle).to(ctx.in_dtype)
+                return grad_x, (gw.to(wdt) if need_w else None), (gb.to(bdt) if need_b else None), None, None
+
+        lib = _lib.load()
+        mean_gxn, dot = torch.empty((2, *std.shape), dtype=torch.float32, device=dev).unbind(0)
         gw = torch.empty(cols, dtype=gdt, device=dev) if need_w else None
         gb = torch.empty(cols, dtype=gdt, device=dev) if need_b else None
         ws_bytes = int(lib.jg_ln_bwd_workspace_bytes(rows, cols)) if (need_w or need_b) else 0
@@ -146,7 +171,7 @@ class _LayerNorm(PositionalFunction):
         _lib.check(rc, "jg_ln_partial_bwd2")
 
         grad_x = None
-        if ctx.needs_input_grad[0]:
+        if need_x:
             _all_reduce(mean_gxn, "avg", group)
             _all_reduce(dot, "sum", group)
             grad_x = torch.empty_like(g)

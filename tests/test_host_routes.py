@@ -87,3 +87,70 @@ def test_native_and_python_route_of_a_step_agree_bit_for_bit(case, monkeypatch):
     assert len(native) == len(python)
     for a, c in zip(native, python):
         assert a.shape == c.shape and a.dtype == c.dtype and torch.equal(a, c)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_norms_and_rings_by_the_native_and_the_python_route_agree_bit_for_bit(dtype, monkeypatch):
+    from jigsaw_amd import attention, groupnorm, layernorm
+
+    dev = torch.device("cuda:0")
+
+    class Half:  # a channel group of two whose other half is the same rows
+        def size(self):
+            return 2
+
+        def all_reduce(self, t, op):
+            if op == "sum":
+                t.mul_(2)
+
+    def leaf(*shape):
+        return torch.randn(*shape, device=dev, generator=gen).to(dtype).requires_grad_()
+
+    def steps():
+        res = []
+        for group, bias in ((None, True), (Half(), True), (Half(), False)):
+            x, w, b = leaf(3, 37, 72), leaf(72), leaf(72) if bias else None
+            y, x_norm, _, var = layernorm._LayerNorm.apply(x, w, b, group, 1e-5)
+            res += [y, x_norm, var, *torch.autograd.grad(y, [t for t in (x, w, b) if t is not None], torch.ones_like(y) * x)]
+            res += [layernorm.layer_norm(x, w, b, group).detach()]
+        for affine in (True, False):
+            x, w, b = leaf(2, 12, 9, 11), leaf(12) if affine else None, leaf(12) if affine else None
+            y = groupnorm.group_norm(x, 3, w, b)
+            res += [y, *torch.autograd.grad(y, [t for t in (x, w, b) if t is not None], torch.ones_like(y) * x)]
+        for shape, sk, P in (((2, 3, 70, 32), 50, 3), ((1, 2, 128, 64), 128, 2)):
+            q, ks, vs = leaf(*shape), [leaf(*shape[:2], sk, shape[3]) for _ in range(P)], [leaf(*shape[:2], sk, shape[3]) for _ in range(P)]
+            out, lse = attention.ring_forward(q, ks, vs, 0.3, rank=1)
+            dq, dk, dv = attention.ring_backward(leaf(*shape), q, out, lse, ks, vs, 0.3)
+            assert not out.requires_grad and not dq.requires_grad
+            res += [out, lse, dq, *dk, *dv]
+        return res
+
+    gen = torch.Generator(device=dev).manual_seed(5)
+    native = steps()
+    monkeypatch.setattr(_lib, "host", lambda: None)
+    gen = torch.Generator(device=dev).manual_seed(5)
+    python = steps()
+    assert len(native) == len(python)
+    for a, c in zip(native, python):
+        assert a.shape == c.shape and a.dtype == c.dtype and a.is_contiguous() == c.is_contiguous() and torch.equal(a, c)
+
+
+@pytest.mark.gpu
+def test_the_native_route_declines_what_needs_a_copy():
+    host, dev = _lib.host(), torch.device("cuda:0")
+    stream = _lib.stream_handle(dev)
+    q = torch.randn(2, 3, 64, 64, device=dev).bfloat16()
+    k = [torch.randn(2, 3, 32, 64, device=dev).bfloat16()]
+    assert host.ring_forward(q, k, k, 1.0, stream) is not None
+    odd = torch.empty(q.numel() + 1, dtype=q.dtype, device=dev)[1:].view_as(q)  # not on a 16-byte boundary
+    for bad_q, bad_k in ((q.transpose(1, 2), k), (odd, k), (q.float(), k), (q, [k[0].half()]), (q, []), (q, k * 17), (q[0], k),
+                         (q[..., :36].contiguous(), [k[0][..., :36].contiguous()]), (q, [k[0][:, :2]])):
+        assert host.ring_forward(bad_q, bad_k, bad_k, 1.0, stream) is None
+        assert host.ring_backward(q, bad_q, q, torch.zeros(2, 3, 64, device=dev), bad_k, bad_k, 1.0, stream) is None
+    assert host.ring_backward(q, q, q, torch.zeros(2, 3, 64, device=dev).half(), k, k, 1.0, stream) is None
+    assert host.ring_forward(torch.zeros(1, 1, 4096, 32, device=dev).bfloat16(), [torch.zeros(1, 1, 4096, 32, device=dev).bfloat16()] * 2,
+                             [torch.zeros(1, 1, 4096, 32, device=dev).bfloat16()] * 2, 1.0, stream) is None  # better off as 64 columns
+    x = torch.randn(4, 6, device=dev)
+    assert host.ln_partial(x.t(), False, stream) is None and host.ln_partial(x.double(), False, stream) is None
+    assert host.gn_forward(x.half(), 2, torch.ones(6, device=dev), None, 1e-5, False, stream) is None  # another type
