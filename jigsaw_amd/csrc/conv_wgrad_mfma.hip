@@ -311,9 +311,18 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
                         2 * ((ptrdiff_t)((size_t)n * p.cin_total * p.Din * plane_x) + (ptrdiff_t)id0 * (ptrdiff_t)plane_x +
                              (ptrdiff_t)ih0 * p.Win + iw0);
     // (with LEAD the window's last dword holds one pixel more than is used; it shares its dword with one that is)
+    const bool rows_inside = oh0 + SR <= p.Hout && ih0 >= 0 && ih0 + NEW <= p.Hin && id0 >= 0 && id0 + KD <= p.Din;
+    // All that a stage's loads of x and g reach lies inside the tensors, whatever columns the rows have
+    constexpr bool kWhole = !FRAMED && CXB != 3;  // (built where there are registers for it)
+    auto whole = [&]() {
+      const char* const x_last = x_org + 2 * ((size_t)(cin_valid - 1) * x_cs + (size_t)(KD - 1) * plane_x + (size_t)(NEW - 1) * p.Win) + 2 * 64 + 16;
+      const char* const g_last = g_org + 2 * ((size_t)(cout_valid - 1) * g_cs + (size_t)(SR - 1) * p.Wout) + 2 * SW + 8;
+      return kWhole && rows_inside && x_org >= reinterpret_cast<const char*>(p.x) && x_last <= p.x_end && g_last <= p.g_end;
+    };
+    // (at stride 2 the window's last pixel is read and not used: a tile that holds one halo column ends before it)
     const bool inside = ALLIN || (oh0 + SR <= p.Hout && ow0 + SW <= p.Wout && ih0 >= 0 &&
-                        ih0 + NEW <= p.Hin && iw0 >= 0 && iw0 + 66 + LEAD <= p.Win && id0 >= 0 &&
-                        id0 + KD <= p.Din);
+                        ih0 + NEW <= p.Hin && iw0 >= 0 && (iw0 + 66 + LEAD <= p.Win || (ST == 2 && iw0 + 65 <= p.Win && whole())) &&
+                        id0 >= 0 && id0 + KD <= p.Din);
     sg.masked = !inside;
     sg.odd = 0;
     if (FRAMED && inside) {
@@ -404,7 +413,6 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
         const int first = max(0, min(count, -col)), past = max(0, min(count, cols - col));
         return ((1u << past) - 1u) & ~((1u << first) - 1u);
       };
-      const uintptr_t safe = reinterpret_cast<uintptr_t>(p.part);
       const int c8 = tid & 7;  // a round is a multiple of 8 chunks: the same in all of them
       sg.g_cols = columns(ow0 + (tid % G_CPR) * 8, 8, p.Wout);
       sg.x_cols = columns(iw0 + c8 * 8, 8, p.Win);
@@ -412,31 +420,41 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
       sg.over = 0;
       sg.g_org = g_org;
       sg.x_org = x_org;
+      // Where only the columns stick out and what is read past them is the tensors' all the same (every strip at the end of
+      // the rows but for its ends), nothing but these masks differs from a stage inside. The workgroups on such a strip
+      // are the last ones to end: 2 x 40 -> 72 channels of 216 x 318 41 -> 37.4 us, of
+      // 217 x 301 48.3 -> 44.6; 4 x 64 -> 128 of 256 x 256 at stride 2, whose padded rows are 257 pixels, 48.6 -> 41.4.
+      if (whole()) {
+        sg.rows = ~0u;
+        sg.tail_cols = has_tail ? columns(iw0 + 64, 2 + 2 * LEAD, p.Win) : 0u;
+      } else {
+        const uintptr_t safe = reinterpret_cast<uintptr_t>(p.part);
 #pragma unroll
-      for (int rd = 0; rd < ROUNDS; ++rd) {
-        const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;
-        const int q = tid + rd * THREADS;
-        bool row_ok;
-        if (g_round) {
-          row_ok = oh0 + (q / G_CPR) % SR < p.Hout;
-        } else {
-          const int rr = (q - G_CHUNKS) / X_CPR;
-          const int row = ih0 + rr % NEW, dd = id0 + (rr / NEW) / CIN_B;
-          row_ok = q < CHUNKS && row >= 0 && row < p.Hin && dd >= 0 && dd < p.Din;
+        for (int rd = 0; rd < ROUNDS; ++rd) {
+          const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;
+          const int q = tid + rd * THREADS;
+          bool row_ok;
+          if (g_round) {
+            row_ok = oh0 + (q / G_CPR) % SR < p.Hout;
+          } else {
+            const int rr = (q - G_CHUNKS) / X_CPR;
+            const int row = ih0 + rr % NEW, dd = id0 + (rr / NEW) / CIN_B;
+            row_ok = q < CHUNKS && row >= 0 && row < p.Hin && dd >= 0 && dd < p.Din;
+          }
+          const bool need = row_ok && (g_round ? sg.g_cols : sg.x_cols) != 0u;
+          const bool fits = at[rd] >= reinterpret_cast<uintptr_t>(g_round ? p.g : p.x) &&
+                            at[rd] + 16 <= reinterpret_cast<uintptr_t>(g_round ? p.g_end : p.x_end);
+          sg.rows |= (need ? 1u : 0u) << rd;
+          sg.over |= (need && !fits ? 1u : 0u) << rd;
+          at[rd] = need && fits ? at[rd] : safe;
         }
-        const bool need = row_ok && (g_round ? sg.g_cols : sg.x_cols) != 0u;
-        const bool fits = at[rd] >= reinterpret_cast<uintptr_t>(g_round ? p.g : p.x) &&
-                          at[rd] + 16 <= reinterpret_cast<uintptr_t>(g_round ? p.g_end : p.x_end);
-        sg.rows |= (need ? 1u : 0u) << rd;
-        sg.over |= (need && !fits ? 1u : 0u) << rd;
-        at[rd] = need && fits ? at[rd] : safe;
+        const int row = ih0 + tid % NEW, dd = id0 + (tid / NEW) / CIN_B;
+        const bool ok = has_tail && dd >= 0 && dd < p.Din && row >= 0 && row < p.Hin;
+        sg.tail_cols = ok ? columns(iw0 + 64, 2 + 2 * LEAD, p.Win) : 0u;
+        const bool fits = t_at >= reinterpret_cast<uintptr_t>(p.x) && t_at + 4 + 4 * LEAD <= reinterpret_cast<uintptr_t>(p.x_end);
+        sg.over |= (sg.tail_cols != 0u && !fits ? 1u : 0u) << 31;
+        t_at = sg.tail_cols != 0u && fits ? t_at : safe;
       }
-      const int row = ih0 + tid % NEW, dd = id0 + (tid / NEW) / CIN_B;
-      const bool ok = has_tail && dd >= 0 && dd < p.Din && row >= 0 && row < p.Hin;
-      sg.tail_cols = ok ? columns(iw0 + 64, 2 + 2 * LEAD, p.Win) : 0u;
-      const bool fits = t_at >= reinterpret_cast<uintptr_t>(p.x) && t_at + 4 + 4 * LEAD <= reinterpret_cast<uintptr_t>(p.x_end);
-      sg.over |= (sg.tail_cols != 0u && !fits ? 1u : 0u) << 31;
-      t_at = sg.tail_cols != 0u && fits ? t_at : safe;
     }
 #pragma unroll
     for (int rd = 0; rd < ROUNDS; ++rd) {

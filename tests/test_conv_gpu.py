@@ -817,3 +817,21 @@ def test_fused_dgrad_fold_any_channels_types_and_strides(case, dtype, dev):
     assert torch.equal(gx.view(bits), halo_fold(want, {}, geom).view(bits))
     for o in offs:
         assert torch.equal(send[o].view(bits), (want_send[o] + 0).view(bits)), f"strip {o}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [
+    # batch, c_in, c_out, padded size, stride: row ends inside a stage's window, with the tensors' ends behind them and not
+    (1, 32, 32, (33, 65), 2), (2, 40, 24, (9, 129), 2), (1, 64, 128, (17, 257), 2), (1, 16, 16, (5, 66), 2), (1, 16, 16, (6, 64), 2),
+    (1, 16, 16, (34, 130), 1), (2, 24, 72, (10, 131), 1), (1, 70, 40, (7, 68), 1), (1, 8, 8, (4, 65), 1),
+], ids=str)
+def test_weight_gradient_at_the_ends_of_rows(case, dtype, dev):
+    """Integers small enough for every sum to be exact: the kernel's result is the exact one, rounded once."""
+    N, ci, co, size, stride = case
+    gen = torch.Generator().manual_seed(6)
+    out = tuple((s - 3) // stride + 1 for s in size)
+    x = torch.randint(-3, 4, (N, ci, *size), generator=gen).double()
+    g = torch.randint(-3, 4, (N, co, *out), generator=gen).double()
+    want = torch.nn.grad.conv2d_weight(x, (co, ci, 3, 3), g, stride=stride)
+    gw, gb = jc.conv_nd_weight(x.to(dtype).to(dev), (co, ci, 3, 3), g.to(dtype).to(dev), stride=stride, with_bias_grad=True)
+    assert torch.equal(gw.cpu(), want.to(dtype)) and torch.equal(gb.cpu(), g.sum((0, 2, 3)).to(dtype))
