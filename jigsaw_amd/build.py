@@ -45,7 +45,7 @@ HIPCC_FLAGS = [
 # v_accvgpr_write around every such use (64 moves per loop iteration in the wide attention forward).
 PER_FILE_FLAGS = {
     name: ["-mllvm", "-amdgpu-mfma-vgpr-form"]
-    for name in ("attn_wide.hip", "attn_swin.hip", "attn_window.hip", "attn_f32_mfma.hip", "proj_mfma.hip")
+    for name in ("attn_wide.hip", "attn_swin.hip", "attn_window.hip", "attn_f32_mfma.hip", "conv_f32.hip", "proj_mfma.hip")
 }
 
 

@@ -45,6 +45,7 @@ bool known(int dt) { return dt == JG_F32 || dt == JG_BF16 || dt == JG_F16; }
 extern "C" size_t jg_conv_workspace_bytes(const jg_conv_desc* desc, int op, int dtype) {
   jg::ConvGeom g;
   if (jg::resolve_conv(desc, "jg_conv_workspace_bytes", &g) != JG_OK) return 0;
+  if (jg::f32_conv_supported(g, dtype)) return op == JG_CONV_WGRAD ? jg::f32_wgrad_workspace(g) : 0;
   switch (op) {
     case JG_CONV_FWD:
       return jg::mfma_fwd_supported(g, dtype) ? jg::mfma_fwd_workspace(g, dtype) : 0;
@@ -67,6 +68,7 @@ extern "C" int jg_conv_fwd(void* y, const void* x, const void* w, const void* bi
   JG_REQUIRE(y && x && w, "jg_conv_fwd: NULL pointer");
   JG_REQUIRE(known(dtype), "jg_conv_fwd: unknown dtype %d", dtype);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (jg::f32_conv_supported(g, dtype)) return jg::f32_fwd(y, x, w, bias, g, s);
   if (jg::mfma_fwd_supported(g, dtype)) return jg::mfma_fwd(y, x, w, bias, g, workspace, workspace_bytes, s, dtype);
   return jg::direct_fwd(y, x, w, bias, g, dtype, s);
 }
@@ -79,6 +81,7 @@ extern "C" int jg_conv_dgrad(void* gx, const void* w, const void* go, const jg_c
   JG_REQUIRE(gx && w && go, "jg_conv_dgrad: NULL pointer");
   JG_REQUIRE(known(dtype), "jg_conv_dgrad: unknown dtype %d", dtype);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (jg::f32_conv_supported(g, dtype)) return jg::f32_dgrad(gx, nullptr, nullptr, nullptr, w, go, g, s);
   if (jg::mfma_dgrad_supported(g, dtype)) return jg::mfma_dgrad(gx, w, go, g, workspace, workspace_bytes, s, dtype);
   return jg::direct_dgrad(gx, w, go, g, dtype, s);
 }
@@ -101,6 +104,7 @@ extern "C" int jg_conv_dgrad_fold(void* gx, void* const send[27], const void* w,
                "jg_conv_dgrad_fold: axis %d: lo %d + size %d + hi %d != padded extent %d", a, lo[a], n[a],
                geom->hi[a], g.in[a]);
   }
+  if (jg::f32_conv_supported(g, dtype)) return jg::f32_dgrad(gx, send, lo, n, w, go, g, static_cast<hipStream_t>(stream));
   if (!jg::mfma_dgrad_supported(g, dtype))
     JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_dgrad_fold: geometry / dtype only has the unfused path");
   return jg::mfma_dgrad_fold(gx, send, lo, n, w, go, g, workspace, workspace_bytes,
@@ -115,6 +119,7 @@ extern "C" int jg_conv_wgrad(void* gw, const void* x, const void* go, const jg_c
   JG_REQUIRE(gw && x && go, "jg_conv_wgrad: NULL pointer");
   JG_REQUIRE(known(dtype), "jg_conv_wgrad: unknown dtype %d", dtype);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (jg::f32_conv_supported(g, dtype)) return jg::f32_wgrad(gw, nullptr, x, go, g, workspace, workspace_bytes, s);
   if (jg::mfma_wgrad_supported(g, dtype))
     return jg::mfma_wgrad(gw, nullptr, x, go, g, workspace, workspace_bytes, s, nullptr, nullptr, nullptr, dtype);
   return jg::direct_wgrad(gw, x, go, g, dtype, workspace, workspace_bytes, s);
@@ -202,6 +207,7 @@ extern "C" int jg_conv_wgrad_bias(void* gw, void* gb, const void* x, const void*
   if (rc) return rc;
   JG_REQUIRE(gw && gb && x && go, "jg_conv_wgrad_bias: NULL pointer");
   JG_REQUIRE(known(dtype), "jg_conv_wgrad_bias: unknown dtype %d", dtype);
+  if (jg::f32_conv_supported(g, dtype)) return jg::f32_wgrad(gw, gb, x, go, g, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
   if (!jg::mfma_wgrad_supported(g, dtype))
     JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_wgrad_bias: geometry only has the separate kernels");
   return jg::mfma_wgrad(gw, gb, x, go, g, workspace, workspace_bytes, static_cast<hipStream_t>(stream), nullptr, nullptr, nullptr,

@@ -835,3 +835,36 @@ def test_weight_gradient_at_the_ends_of_rows(case, dtype, dev):
     want = torch.nn.grad.conv2d_weight(x, (co, ci, 3, 3), g, stride=stride)
     gw, gb = jc.conv_nd_weight(x.to(dtype).to(dev), (co, ci, 3, 3), g.to(dtype).to(dev), stride=stride, with_bias_grad=True)
     assert torch.equal(gw.cpu(), want.to(dtype)) and torch.equal(gb.cpu(), g.sum((0, 2, 3)).to(dtype))
+
+
+@pytest.mark.parametrize("case", [
+    # batch, c_in, c_out, size of x, padding: 8 x 64 tiles of the outputs (4 x 64 in the weight gradient), stages of 8 channels, blocks of
+    # 16 and 32 produced channels, 7 or 14 input channels of the weight gradient, rows that are whole cache lines
+    (1, 1, 1, (3, 3), (0, 0)), (2, 3, 16, (10, 66), (0, 0)), (1, 3, 17, (11, 67), (0, 0)), (2, 2, 33, (9, 65), (1, 1)), (1, 7, 5, (8, 64), (2, 2)),
+    (2, 8, 32, (8, 128), (1, 1)), (1, 9, 15, (17, 129), (0, 1)), (3, 14, 16, (5, 40), (2, 0)), (1, 15, 65, (12, 96), (1, 1)), (1, 70, 4, (18, 70), (1, 0)),
+    (2, 64, 64, (24, 33), (0, 0)), (1, 33, 63, (40, 100), (1, 1)), (5, 12, 12, (70, 200), (0, 0)),
+], ids=str)
+def test_fp32_on_the_matrix_instruction(case, dev):
+    """Integers: every sum is exact, so are the results. Then no result further from float64's than its longest chain of fp32 additions allows:
+    nine taps of a stage's 8 channels and the stages; eight pixels, then doubles, and two roundings to fp32, in the weight gradient."""
+    N, ci, co, size, pad = case
+    gen = torch.Generator().manual_seed(7)
+    out = tuple(s + 2 * p - 2 for s, p in zip(size, pad))
+    shapes = (N, ci, *size), (co, ci, 3, 3), (co,), (N, co, *out)
+
+    def check(x, w, b, g, chain_y, chain_x, chain_w):
+        y = jc.conv_nd(*(t.float().to(dev) for t in (x, w, b)), padding=pad)
+        gx = jc.conv_nd_input(x.shape, w.float().to(dev), g.float().to(dev), padding=pad)
+        gw, gb = jc.conv_nd_weight(x.float().to(dev), w.shape, g.float().to(dev), padding=pad, with_bias_grad=True)
+        f, fx, fw = torch.nn.functional.conv2d, torch.nn.grad.conv2d_input, torch.nn.grad.conv2d_weight
+        a = [t.abs() for t in (x, w, b, g)]
+        for name, got, want, size_of, chain in (
+                ("y", y, f(x, w, b, padding=pad), f(a[0], a[1], a[2], padding=pad), chain_y),
+                ("gx", gx, fx(x.shape, w, g, padding=pad), fx(x.shape, a[1], a[3], padding=pad), chain_x),
+                ("gw", gw, fw(x, w.shape, g, padding=pad), fw(a[0], w.shape, a[3], padding=pad), chain_w),
+                ("gb", gb, g.sum((0, 2, 3)), a[3].sum((0, 2, 3)), chain_w)):
+            off = (got.cpu().double() - want).abs() - chain * 2.0**-24 * size_of
+            assert off.max() <= 0, f"{name}: {off.max()}"
+
+    check(*(torch.randint(-3, 4, s, generator=gen).double() for s in shapes), 0, 0, 0)
+    check(*(torch.randn(s, generator=gen).double() for s in shapes), 74 + ci // 8, 74 + co // 8, 12)
