@@ -61,6 +61,7 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -1171,11 +1172,11 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
 
   // The same for any type and number of channels, and for the strided gradient (a lane's two phases are the pixels ow and
   // ow + 1). One store a pixel (two neighbours of the strided gradient together) and channel, as the epilogues for such
-  // rows have it; bound by the latency of a workgroup's few stages and these stores. It takes 8 to 18 us more than the plain
+  // rows have it; bound by the latency of a workgroup's few stages and these stores. It takes 2 to 20 us more than the plain
   // epilogue at the sizes below, and saves writing the padded gradient, its pack and its fold: gradient to finished fold of
-  // 2 x 72 -> 40 channels of 217 x 301 bf16 56 -> 53 us, of 4 x 128 -> 64 of 256 x 256 at stride 2 72 -> 67 us, of
-  // 4 x 16 -> 3 of 256 x 256 fp32 47 -> 43 us, each with one launch less.
-  auto epilogue_fold_any = [&](const TileCoord& tc) {
+  // 2 x 72 -> 40 channels of 217 x 301 bf16 56 -> 47 us, at stride 2 of 4 x 128 -> 64 of 256 x 256 72 -> 59 us and of
+  // 8 x 99 -> 123 of 218 x 162 143 -> 122 us, of 2 x 79 -> 53 of 212 x 41 fp32 128 -> 127 us, each with one launch less.
+  auto epilogue_fold_any = [&](const TileCoord& tc, int free_buf) {
     // The parameters as they are in the kernel-argument segment, read here: held in scalar registers from the kernel's
     // start on they push the stage loop's own out of them.
     typedef const __attribute__((address_space(4))) FwdParams* Args;
@@ -1199,14 +1200,35 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     const int hi_h = Hp - p.lo_h - p.nH, hi_w = Wp - p.lo_w - p.nW;
     const int rw0 = region(ow, p.lo_w, p.nW), rw1 = region(ow + 1, p.lo_w, p.nW);
     const bool in0 = ow >= 0 && ow < Wp, in1 = PHASES && ow + 1 >= 0 && ow + 1 < Wp;
-    // Values pass through `0 + v`, as in epilogue_fold: the sign of a zero, and of what rounds to one, is cleared
     auto pair16 = [&](float lo, float hi) {
       f32x2 v2 = {lo, hi};
-      const uint32_t h2 = F16 ? __builtin_bit_cast(uint32_t, __builtin_convertvector(v2, f16x2)) : __builtin_bit_cast(uint32_t, __builtin_convertvector(v2, bf16x2));
-      uint32_t some;  // a one in every half that is not a zero
-      asm("v_pk_min_u16 %0, %1, %2" : "=v"(some) : "v"(h2 & 0x7fff7fffu), "v"(0x00010001u));
-      return h2 & (some << 15 | 0x7fff7fffu);
+      return F16 ? __builtin_bit_cast(uint32_t, __builtin_convertvector(v2, f16x2)) : __builtin_bit_cast(uint32_t, __builtin_convertvector(v2, bf16x2));
     };
+    // The sign of a zero, and of what rounds to one, is cleared, as in epilogue_fold. Such values are rare; as integers they are the
+    // least, so that one min3 per two values finds out (the zeros of channels that do not exist are none of them).
+    const int least_zero = p.out_kind == 1 ? (int)0x80000000u : (F16 ? (int)0xb3000000u : (int)0x80008000u);  // -0, -2^-25, -2^-134
+    int least = 0x7fffffff;
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+      for (int r = 0; r < WROWS; ++r)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float v = acc[cb][r][i];  // (a bit cast of the element itself reads element 0)
+          least = min(least, __builtin_bit_cast(int, v));
+        }
+    if (__builtin_amdgcn_ballot_w64(least <= least_zero) != 0) {
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int r = 0; r < WROWS; ++r)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const float v = acc[cb][r][i];
+            acc[cb][r][i] = __builtin_bit_cast(int, v) <= least_zero ? 0.0f : v;
+          }
+    }
+    unsigned char* const scratch = reinterpret_cast<unsigned char*>(lds_in + free_buf * STAGE_SLOTS) + wave * (STAGE_BYTES / WAVES);
     const int blocks = PHASES ? 1 : CB;
 #pragma unroll
     for (int r = 0; r < WROWS; ++r) {
@@ -1225,8 +1247,8 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
         const uint32_t first = 4 * kg * st + es * (uint32_t)(ow - p.lo_w);
         const bool m0 = in0 && rw0 == 1, m1 = in1 && rw1 == 1;
         if (p.out_kind == 1) {
-          if (m0) walk_channels(blocks, first, st, [&](int cb, int i, uint32_t vo) { store_f32(base, vo, acc[cb][r][i] + 0.0f); });
-          if (m1) walk_channels(blocks, first + 4, st, [&](int, int i, uint32_t vo) { store_f32(base, vo, acc[CB - 1][r][i] + 0.0f); });
+          if (m0) walk_channels(blocks, first, st, [&](int cb, int i, uint32_t vo) { store_f32(base, vo, acc[cb][r][i]); });
+          if (m1) walk_channels(blocks, first + 4, st, [&](int, int i, uint32_t vo) { store_f32(base, vo, acc[CB - 1][r][i]); });
         } else if (!PHASES) {
           if (m0)
             walk_channels(blocks, first, st, [&](int cb, int i, uint32_t vo) {
@@ -1241,23 +1263,45 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
             walk_channels(blocks, m0 ? first : first + 2, st, [&](int, int i, uint32_t vo) { store_bf16_lo(base, vo, m0 ? both(i) : both(i) >> 16); });
         }
       }
-      // The few pixels at the edges, each lane with an address of its own
-      auto edge = [&](bool mine, int at, int rw, auto value) __attribute__((always_inline)) {
-        if (__builtin_amdgcn_ballot_w64(mine) == 0) return;
-        char* const lo = static_cast<char*>(strip_entry(slot0));
-        char* const hi = static_cast<char*>(strip_entry(slot0 + 2));
-        char* const to = rw == 0 ? lo : hi;
-        if (!mine || to == nullptr) return;
-        const uint32_t ew = (uint32_t)(rw == 0 ? p.lo_w : hi_w), pe = (uint32_t)ed * (uint32_t)eh * ew;
-        const int cw = rw == 0 ? at : at - p.lo_w - p.nW;
-        const uintptr_t d = reinterpret_cast<uintptr_t>(to) + es * ((plane0 + 4 * kg) * (size_t)pe + (size_t)(cd * eh + ch) * ew + cw);
-        walk_channels(blocks, 0u, es * pe, [&](int cb, int i, uint32_t vo) {
-          if (p.out_kind == 1) *reinterpret_cast<__attribute__((address_space(1))) float*>(d + vo) = value(cb, i) + 0.0f;
-          else *reinterpret_cast<__attribute__((address_space(1))) uint16_t*>(d + vo) = (uint16_t)pair16(value(cb, i), 0.0f);
-        });
+      // The few pixels at the edges, one after the other: its two lanes lay the channels into LDS, and each lane stores one
+      // (a store per channel with one lane of 64 at work took 17 % of the kernel where half of the tiles have an edge)
+      auto edge = [&](bool mine, int at, auto value) __attribute__((always_inline)) {
+        for (uint32_t todo = (uint32_t)__builtin_amdgcn_ballot_w64(mine); todo != 0; todo &= todo - 1) {
+          const int src = __builtin_ctz(todo), col = __builtin_amdgcn_readlane(at, src);
+          const bool low = col < p.lo_w;
+          char* const to = static_cast<char*>(strip_entry(slot0 + (low ? 0 : 2)));
+          if (to == nullptr) continue;
+          if (ln == src) {
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+              if (cb >= blocks) break;
+              unsigned char* const to4 = scratch + es * (cb * 32 + 4 * kg);  // channels cb * 32 + 2 i + 4 kg + 0..3
+              if (p.out_kind == 1) {
+#pragma unroll
+                for (int i = 0; i < 16; i += 4)
+                  *reinterpret_cast<f32x4*>(to4 + 8 * i) = f32x4{value(cb, i), value(cb, i + 1), value(cb, i + 2), value(cb, i + 3)};
+              } else {
+#pragma unroll
+                for (int i = 0; i < 16; i += 4)
+                  *reinterpret_cast<u32x2*>(to4 + 4 * i) = u32x2{pair16(value(cb, i), value(cb, i + 1)), pair16(value(cb, i + 2), value(cb, i + 3))};
+              }
+            }
+          }
+          asm volatile("" ::: "memory");  // (a wavefront's own reads and writes of LDS are done in order)
+          const uint32_t ew = (uint32_t)(low ? p.lo_w : hi_w), pe = (uint32_t)ed * (uint32_t)eh * ew;
+          const int cw = low ? col : col - p.lo_w - p.nW;
+          const uintptr_t d = reinterpret_cast<uintptr_t>(to) + es * ((plane0 + lane) * (size_t)pe + (size_t)(cd * eh + ch) * ew + cw);
+          if (lane < min(m_here, 32 * blocks)) {
+            if (p.out_kind == 1)
+              *reinterpret_cast<__attribute__((address_space(1))) uint32_t*>(d) = *reinterpret_cast<const uint32_t*>(scratch + 4 * lane);
+            else
+              *reinterpret_cast<__attribute__((address_space(1))) uint16_t*>(d) = *reinterpret_cast<const uint16_t*>(scratch + 2 * lane);
+          }
+          asm volatile("" ::: "memory");
+        }
       };
-      edge(in0 && rw0 != 1, ow, rw0, [&](int cb, int i) { return acc[cb][r][i]; });
-      if (PHASES) edge(in1 && rw1 != 1, ow + 1, rw1, [&](int, int i) { return acc[CB - 1][r][i]; });
+      edge(in0 && rw0 != 1, ow, [&](int cb, int i) { return acc[cb][r][i]; });
+      if (PHASES) edge(in1 && rw1 != 1, ow + 1, [&](int, int i) { return acc[CB - 1][r][i]; });
     }
   };
 
@@ -1275,12 +1319,12 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   // all six: 1.59 M. (In the fold's epilogue the older wavefronts of a SIMD get their stores out first and are
   // back in the stage loop while 4 to 7 still store.)
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const bool stage_early = FOLD ? (wave_u == 4 || wave_u == 5) : (wave_u == 0 || wave_u == 1);
+  const bool stage_early = FOLD == FOLD_WHOLE ? (wave_u == 4 || wave_u == 5) : (wave_u == 0 || wave_u == 1);
   // Does the epilogue put anything into the free stage buffer? Every epilogue but the fold's does (rows go
   // through LDS to leave as 16-byte pieces), and the fold's does where the tile grid lies on the 16-byte grid
   // of the unpadded gradient (the same test as in epilogue_fold; it is the same for every tile of a launch).
   const bool epilogue_uses_lds =
-      MODE == STRIDED_DGRAD || FOLD == FOLD_ANY ? false : !FOLD || ((((p.org_w - p.lo_w) & 7) == 0) && (p.nW & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
+      FOLD == FOLD_ANY ? true : MODE == STRIDED_DGRAD ? false : !FOLD || ((((p.org_w - p.lo_w) & 7) == 0) && (p.nW & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
   int buf = 0;
   cursor_enter(0);
   issue_stage();
@@ -1346,7 +1390,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     // free until the next stage is stored into it. That store waits (barrier above, in the first
     // stage of the next tile) until every wavefront has left this epilogue; until then a
     // wavefront that is done early already runs the next tile's MFMAs.
-    if constexpr (FOLD == FOLD_ANY) epilogue_fold_any(tcur);
+    if constexpr (FOLD == FOLD_ANY) epilogue_fold_any(tcur, buf ^ 1);
     else if constexpr (FOLD == FOLD_WHOLE) epilogue_fold(tcur, buf ^ 1);
     else epilogue(tcur, buf ^ 1);
   }
