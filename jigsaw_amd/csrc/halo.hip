@@ -946,13 +946,18 @@ __global__ __launch_bounds__(256) void fold_rows_kernel(Table tab,
 
 // In-place second half of a fold: gx already holds `0 + own`; only the cells that a
 // neighbour reaches change. The rows that a D or H neighbour reaches are summed in full,
-// up to a wavefront per row; of the other rows only the first and last columns change, one lane
-// per cell. Both in one launch, the blocks of the rows first: they are few and wait for chains of
-// loads, the columns' blocks for a cache line per cell, and neither fills the chip (8 x 64
-// channels of 1024 x 1024: 66 -> 55 us, 2 x 32 of 128 x 128 x 128 87 -> 72 us; two launches before).
+// up to a wavefront per row, and their first and last columns, which more neighbours reach, one lane per cell; of the
+// other rows only the first and last columns change, one lane per cell. All in one launch, the blocks of the rows first: they
+// are few and wait for loads, the columns' blocks for a cache line per cell, and neither fills the chip (8 x 64
+// channels of 1024 x 1024: 66 -> 55 us, 2 x 32 of 128 x 128 x 128 87 -> 72 us; two launches before). What a lane adds along H
+// and W is loaded before any of it is added; term after term, edge columns and the rest of a row in one lane, 2 x 40 channels of
+// 217 x 301 took 12 us (now 6), 8 x 123 of 218 x 163 21 (12), 32 of 100 x 90 x 77 30 (16). The edge lanes come first: last,
+// behind the columns, they took 14 us more in the volume of 128 x 128 x 128; a load for every term, where there is none from the
+// lane's own cell, 3 us more.
 struct BorderPlan {
   uint32_t rows_per_plane;  // rows of a plane that a D or H neighbour reaches
-  uint32_t row_items, col_items, row_blocks;  // such rows, edge cells of all rows; blocks that take rows
+  uint32_t row_items, edge_items, col_items;  // such rows, their edge cells, edge cells of all rows
+  uint32_t edge_blocks, row_blocks;           // blocks that take those edge cells, and rows
   int nbd, nbh;             // border depths / border rows of a non-border depth
   int n_edge, head;         // W-edge cells of a row: columns [0, head) and [W - lo, W)
   int lpr;                  // lanes per row of the rows kernel
@@ -960,18 +965,11 @@ struct BorderPlan {
 };
 
 
-template <int DT>
-__device__ __forceinline__ void fold_border_rows(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp) {
-  typedef typename Arith<DT>::T T;
-  constexpr int V = Bits<T>::V;
-  // a row is owned by bp.lpr lanes (a power of two up to 64: a whole wavefront for long rows)
-  const uint32_t item = (blockIdx.x * 256u + threadIdx.x) / (uint32_t)bp.lpr;
-  if (item >= bp.row_items) return;
-  const int lane = threadIdx.x & (bp.lpr - 1);
-  const int D = g.n[0], H = g.n[1], W = g.n[2];
+// (plane, d, h) of a row that a D or H neighbour reaches
+__device__ __forceinline__ uint32_t border_row(uint32_t item, const Geom& g, const BorderPlan& bp, int& d, int& h) {
+  const int D = g.n[0], H = g.n[1];
   const uint32_t pp = mdiv(item, bp.div_rows);
   const uint32_t idx = item - pp * bp.rows_per_plane;
-  int d, h;
   if (idx < (uint32_t)bp.nbd * (uint32_t)H) {
     const uint32_t k = mdiv(idx, bp.div_h);
     d = border_coord((int)k, D, g.lo[0], g.hi[0]);
@@ -982,17 +980,126 @@ __device__ __forceinline__ void fold_border_rows(typename Arith<DT>::T* __restri
     d = g.hi[0] + (int)di;
     h = border_coord((int)(idx2 - di * (uint32_t)bp.nbh), H, g.lo[1], g.hi[1]);
   }
-  const long long p = (long long)pp;
-  T* drow = gx + ((p * D + d) * H + h) * (long long)W;
-  const int n_vec = W / V;
-  for (int j = lane; j < n_vec; j += bp.lpr) fold_span<DT>(drow, drow, g, p, d, h, j * V, V);
-  if (lane == 0 && n_vec * V < W) fold_span<DT>(drow, drow, g, p, d, h, n_vec * V, W - n_vec * V);
+  return pp;
+}
+
+// Columns [b, e) of such a row, between the edge columns: parts of the vector [c0, c0 + V) the row is cut into.
+template <int DT>
+__device__ __forceinline__ void fold_border_span(typename Arith<DT>::T* drow, const Geom& g, long long p, int d, int h, int c0, int b, int e) {
+  typedef typename Arith<DT>::T T;
+  constexpr int V = Bits<T>::V;
+  typedef uint32_t u32x4_e __attribute__((ext_vector_type(4), aligned(2)));
+  const bool whole = e - b == V;
+  float acc_d[V] = {};
+#pragma unroll 1
+  for (int od = -1; od <= 1; ++od) {
+    int cd, ed;
+    if (!reach(od, d, g.lo[0], g.n[0], g.hi[0], cd, ed)) continue;
+    T mb[3][V];
+    bool have[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      int ch, eh;
+      const bool in = reach(k - 1, h, g.lo[1], g.n[1], g.hi[1], ch, eh), self = od == 0 && k == 1;
+      const T* const strip = static_cast<const T*>(table_entry((od + 1) * 9 + k * 3 + 1));
+      have[k] = self || (in && strip != nullptr);
+      const T* const from = self ? drow : strip + ((p * ed + cd) * eh + ch) * g.n[2];
+      if (!have[k]) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) mb[k][i] = T(0);
+      } else if (c0 + V <= g.n[2]) {  // (edge cells that another lane changes at the same time are read, not used)
+        const u32x4 v = *reinterpret_cast<const u32x4_e*>(from + c0);
+        __builtin_memcpy(mb[k], &v, 16);
+      } else {
+#pragma unroll
+        for (int i = 0; i < V; ++i) mb[k][i] = from[min(max(c0 + i, b), e - 1)];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      float acc_h = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) acc_h = Arith<DT>::up(Arith<DT>::down(acc_h + Arith<DT>::up(mb[k][i])));
+      acc_d[i] = Arith<DT>::up(Arith<DT>::down(acc_d[i] + acc_h));
+    }
+  }
+  T ob[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) ob[i] = Arith<DT>::down(acc_d[i]);
+  if (whole) {
+    u32x4 out;
+    __builtin_memcpy(&out, ob, 16);
+    *reinterpret_cast<u32x4_e*>(drow + c0) = out;
+  } else {
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      if (c0 + i >= b && c0 + i < e) drow[c0 + i] = ob[i];
+  }
+}
+
+template <int DT>
+__device__ __forceinline__ void fold_border_rows(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp) {
+  typedef typename Arith<DT>::T T;
+  constexpr int V = Bits<T>::V;
+  // a row is owned by bp.lpr lanes (a power of two up to 64: a whole wavefront for long rows)
+  const uint32_t item = ((blockIdx.x - bp.edge_blocks) * 256u + threadIdx.x) / (uint32_t)bp.lpr;
+  if (item >= bp.row_items) return;
+  int d, h;
+  const long long p = (long long)border_row(item, g, bp, d, h);
+  const int W = g.n[2], up0 = W - g.lo[2];
+  T* drow = gx + ((p * g.n[0] + d) * g.n[1] + h) * (long long)W;
+  for (int c0 = (threadIdx.x & (bp.lpr - 1)) * V; c0 < up0; c0 += bp.lpr * V) {
+    const int b = max(c0, bp.head), e = min(c0 + V, up0);
+    if (b < e) fold_border_span<DT>(drow, g, p, d, h, c0, b, e);
+  }
+}
+
+// The edge columns of such a row, one lane per cell
+template <int DT>
+__device__ __forceinline__ void fold_border_edges(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp) {
+  typedef typename Arith<DT>::T T;
+  const uint32_t at = blockIdx.x * 256u + threadIdx.x;
+  if (at >= bp.edge_items) return;
+  const uint32_t item = mdiv(at, bp.div_edge);
+  const int q = (int)(at - item * (uint32_t)bp.n_edge);
+  int d, h;
+  const long long p = (long long)border_row(item, g, bp, d, h);
+  const int W = g.n[2], up0 = W - g.lo[2], c = q < bp.head ? q : up0 + (q - bp.head);
+  T* const cell = gx + ((p * g.n[0] + d) * g.n[1] + h) * (long long)W + c;
+  float acc_d = 0.0f;
+#pragma unroll 1
+  for (int od = -1; od <= 1; ++od) {
+    int cd, ed;
+    if (!reach(od, d, g.lo[0], g.n[0], g.hi[0], cd, ed)) continue;
+    T v[9];
+    bool have[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      int ch, eh, cw, ew;
+      const bool in_h = reach(k / 3 - 1, h, g.lo[1], g.n[1], g.hi[1], ch, eh), in_w = reach(k % 3 - 1, c, g.lo[2], W, g.hi[2], cw, ew);
+      const bool self = od == 0 && k == 4;
+      const T* const strip = static_cast<const T*>(table_entry((od + 1) * 9 + k));
+      have[k] = self || (in_h && in_w && strip != nullptr);
+      v[k] = T(0);
+      if (have[k]) v[k] = *(self ? cell : strip + ((p * ed + cd) * eh + ch) * ew + cw);
+    }
+    float acc_h = 0.0f;
+#pragma unroll
+    for (int kh = 0; kh < 3; ++kh) {
+      float acc_w = 0.0f;
+#pragma unroll
+      for (int kw = 0; kw < 3; ++kw) acc_w = Arith<DT>::up(Arith<DT>::down(acc_w + Arith<DT>::up(v[kh * 3 + kw])));
+      acc_h = Arith<DT>::up(Arith<DT>::down(acc_h + acc_w));
+    }
+    acc_d = Arith<DT>::up(Arith<DT>::down(acc_d + acc_h));
+  }
+  *cell = Arith<DT>::down(acc_d);
 }
 
 template <int DT>
 __device__ __forceinline__ void fold_border_cols(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp) {
   typedef typename Arith<DT>::T T;
-  const uint32_t item = (blockIdx.x - bp.row_blocks) * 256u + threadIdx.x;  // (row, edge cell), cell fastest
+  const uint32_t item = (blockIdx.x - bp.edge_blocks - bp.row_blocks) * 256u + threadIdx.x;  // (row, edge cell), cell fastest
   if (item >= bp.col_items) return;
   const int D = g.n[0], H = g.n[1], W = g.n[2];
   const uint32_t row = mdiv(item, bp.div_edge);
@@ -1001,29 +1108,26 @@ __device__ __forceinline__ void fold_border_cols(typename Arith<DT>::T* __restri
   const int h = (int)(row - t2 * (uint32_t)H);
   const uint32_t pp = mdiv(t2, bp.div_d);
   const int d = (int)(t2 - pp * (uint32_t)D);
-  // rows that a D or H neighbour reaches belong to the other kernel
+  // (not the rows that a D or H neighbour reaches)
   if (!((d >= g.hi[0]) && (d < D - g.lo[0]) && (h >= g.hi[1]) && (h < H - g.lo[1]))) return;
   const int up0 = W - g.lo[2];
   const int c = q < bp.head ? q : up0 + (q - bp.head);
   T* cell = gx + (long long)row * W + c;
-  float acc = 0.0f;
-  if (c < g.hi[2]) {
-    const T* s_lo = static_cast<const T*>(table_entry(9 + 3 + 0));
-    if (s_lo != nullptr) acc = Arith<DT>::up(Arith<DT>::down(acc + Arith<DT>::up(s_lo[(long long)row * g.hi[2] + c])));
-  }
-  acc = Arith<DT>::up(Arith<DT>::down(acc + Arith<DT>::up(*cell)));
-  if (c >= up0) {
-    const T* s_hi = static_cast<const T*>(table_entry(9 + 3 + 2));
-    if (s_hi != nullptr)
-      acc = Arith<DT>::up(Arith<DT>::down(acc + Arith<DT>::up(s_hi[(long long)row * g.lo[2] + (c - up0)])));
-  }
+  const T* const s_lo = static_cast<const T*>(table_entry(9 + 3 + 0));
+  const T* const s_hi = static_cast<const T*>(table_entry(9 + 3 + 2));
+  const bool lower = c < g.hi[2] && s_lo != nullptr, upper = c >= up0 && s_hi != nullptr;
+  const T own = *cell, v_lo = *(lower ? s_lo + (long long)row * g.hi[2] + c : cell), v_hi = *(upper ? s_hi + (long long)row * g.lo[2] + (c - up0) : cell);
+  float acc = lower ? Arith<DT>::up(Arith<DT>::down(0.0f + Arith<DT>::up(v_lo))) : 0.0f;
+  acc = Arith<DT>::up(Arith<DT>::down(acc + Arith<DT>::up(own)));
+  if (upper) acc = Arith<DT>::up(Arith<DT>::down(acc + Arith<DT>::up(v_hi)));
   *cell = Arith<DT>::down(acc);
 }
 
 // tab comes first among the parameters: its entries are read from the kernel-argument segment
 template <int DT>
 __global__ __launch_bounds__(256) void fold_border_kernel(Table tab, typename Arith<DT>::T* __restrict__ gx, Geom g, BorderPlan bp) {
-  if (blockIdx.x < bp.row_blocks) fold_border_rows<DT>(gx, g, bp);
+  if (blockIdx.x < bp.edge_blocks) fold_border_edges<DT>(gx, g, bp);
+  else if (blockIdx.x < bp.edge_blocks + bp.row_blocks) fold_border_rows<DT>(gx, g, bp);
   else fold_border_cols<DT>(gx, g, bp);
 }
 
@@ -1378,15 +1482,17 @@ template <int DT>
 bool launch_border(const Table& tab, void* gx, const Geom& g, BorderPlan bp, unsigned long long row_items,
                    unsigned long long col_items, hipStream_t s) {
   typedef typename Arith<DT>::T T;
-  const int vecs = g.n[2] / (16 / (int)sizeof(T));
+  const int V = 16 / (int)sizeof(T), vecs = (g.n[2] - g.lo[2] + V - 1) / V;
   bp.lpr = 1;
   while (bp.lpr < 64 && bp.lpr < vecs) bp.lpr *= 2;
-  const unsigned long long threads = row_items * (unsigned long long)bp.lpr;
-  if (threads >= (1ull << 32) || col_items >= (1ull << 32)) return false;
+  const unsigned long long threads = row_items * (unsigned long long)bp.lpr, edge_items = row_items * (unsigned long long)bp.n_edge;
+  if (threads >= (1ull << 32) || edge_items >= (1ull << 31) || col_items >= (1ull << 32)) return false;
+  bp.edge_items = (uint32_t)edge_items;
+  bp.edge_blocks = (uint32_t)((edge_items + 255) / 256);
   bp.row_items = (uint32_t)row_items;
   bp.col_items = (uint32_t)col_items;
   bp.row_blocks = (uint32_t)((threads + 255) / 256);
-  const unsigned long long blocks = bp.row_blocks + (col_items + 255) / 256;
+  const unsigned long long blocks = bp.edge_blocks + bp.row_blocks + (col_items + 255) / 256;
   if (blocks == 0) return true;
   fold_border_kernel<DT><<<(unsigned)blocks, 256, 0, s>>>(tab, static_cast<T*>(gx), g, bp);
   return true;

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from helpers import assert_bit_equal, conv_geometry, mesh_coords, neighbour, special_values_
-from jigsaw_amd.halo import HaloGeometry, halo_assemble, halo_fold, halo_pack
+from jigsaw_amd.halo import HaloGeometry, halo_assemble, halo_fold, halo_fold_border_, halo_pack
 from oracle import halo as oh
 
 pytestmark = pytest.mark.gpu
@@ -89,6 +89,32 @@ def test_fold_matches_oracle_bitwise(case, dtype, dev):
     for c in mesh_coords(mesh):
         strips = gpu_strips(grads_gpu, geoms, c, mesh, from_padded=True)
         got = halo_fold(grads_gpu[c], strips, geoms[c])
+        assert_bit_equal(got, want[c], f"rank {c}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [c for c in CASES if min(c[0]) > 1] + [
+    # rows of one vector and its neighbours, halos that leave nothing between the edge columns, odd rows, several rounds of a wavefront
+    ((3, 3), (3, 4), (3, 3), (1, 1), (1, 1), (1, 1)), ((2, 3), (2, 7), (3, 7), (1, 1), (1, 3), (1, 1)), ((3, 3), (5, 10), (3, 3), (1, 1), (1, 1), (1, 1)),
+    ((3, 2), (3, 301), (3, 3), (1, 1), (1, 1), (1, 1)), ((2, 2, 3), (3, 4, 17), (3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1)),
+    ((3, 3, 2), (2, 3, 9), (5, 3, 3), (1, 1, 1), (2, 1, 1), (1, 1, 1)),
+], ids=_case_id)
+def test_fold_in_place_matches_oracle_bitwise(case, dtype, dev):
+    """The own part first, the neighbours' blocks added in place: the oracle's bits."""
+    mesh, n, k, s, p, d = case
+    torch.manual_seed(2)
+    geoms = {c: conv_geometry(n, mesh, c, k, s, p, d) for c in mesh_coords(mesh)}
+    grads = {}
+    for c, g in geoms.items():
+        t = torch.randn(2, 3, *g.padded) * torch.exp2(torch.randint(-12, 12, (2, 3, *g.padded)).float())
+        grads[c] = special_values_(t).to(dtype)
+    want = oh.scatter_add_mesh(grads, mesh, k, s, p, d, n)
+    grads_gpu = {c: t.to(dev) for c, t in grads.items()}
+    for c in mesh_coords(mesh):
+        if not geoms[c].same_on_every_rank:
+            continue  # their blocks have widths of their own: halo_fold does that
+        got = halo_fold(grads_gpu[c], {}, geoms[c])
+        halo_fold_border_(got, gpu_strips(grads_gpu, geoms, c, mesh, from_padded=True), geoms[c])
         assert_bit_equal(got, want[c], f"rank {c}")
 
 
