@@ -379,14 +379,12 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
 constexpr int DKV_STATS = 2 * BT * 4;                 // lse2[64], delta[64] as floats
 constexpr int DKV_HALF = 2 * NAT + DKV_STATS;         // Q tile, dO tile + stats
 constexpr int DKV_LDS = 4 * DKV_HALF;                 // 67584: two query halves, double buffered
-// Key blocks per workgroup. With 2 (4 wavefronts, 64 keys) a launch has twice the workgroups, two of
-// which share a CU: the two wavefronts of a SIMD then belong to different workgroups and do not
-// march in step (the barrier per tile keeps the wavefronts of ONE workgroup in the same phase:
-// all in their matrix instructions, then all in their exponentials).
-#ifndef JG_DKV_KB
-#define JG_DKV_KB 4
-#endif
-constexpr int DKV_KB = JG_DKV_KB;
+// Key blocks per workgroup: 2 (4 wavefronts, 64 keys), so that two workgroups share a CU. The two wavefronts of a SIMD then belong to
+// different workgroups and do not march in step (the barrier per tile keeps the wavefronts of ONE workgroup in the same phase: all
+// in their matrix instructions, then all in their exponentials), and a small launch fills more of the chip. With 4 (8 wavefronts) : 2,
+// us: 24 heads x 2 chunks of 1000 46 : 37, 8 x 4 of 4096 327 : 311, 64 x 1 of 4096 625 : 572, 3 x 2 of 1497 28 : 20, 4 x 2 of 128
+// 8.2 : 5.7, 16 x 1 of 2048 45 : 43; nothing slower.
+constexpr int DKV_KB = 2;
 constexpr int DKV_THREADS = 64 * 2 * DKV_KB;
 constexpr int DKV_ROWS = 32 * DKV_KB;                 // keys per workgroup
 constexpr int DKV_SHARE = BT / DKV_KB;                // rows of a streamed tile each wavefront of a half moves
