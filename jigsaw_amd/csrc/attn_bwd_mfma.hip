@@ -20,9 +20,9 @@
 //   5 of a one-kernel formulation) so that P / dS are always produced in the
 //   register layout the next MFMA consumes and never travel through LDS.
 //
-//   Workgroup: 512 threads = 8 wavefronts = 4 blocks of 32 rows (queries for dQ,
-//   keys for dK/dV) x 2 halves of the streamed side, combined through LDS.
-//   Streamed tiles (64 rows x 128 bytes) travel from memory straight into LDS, row-major
+//   Workgroup: 8 wavefronts (dQ: 4 in small launches; dK/dV: 4) = 4 or 2 blocks of 32 rows (queries
+//   for dQ, keys for dK/dV) x 2 halves of the streamed side, combined through LDS.
+//   Streamed tiles (64 rows x 128 bytes; 32 rows where dQ has 2 blocks) travel from memory straight into LDS, row-major
 //   with the 16-byte chunks of a row XOR-swizzled by row % 8 (no registers, no vector
 //   instructions, no second, transposed copy): the transposed fragments come from
 //   ds_read_b64_tr_b16 (within 16 lanes, lane i receives element i % 4 of the 8 bytes
@@ -42,6 +42,8 @@
 //   jigsaw/modules/attention/_functional/cores/math.py:125-149
 #include "attn_chunks.h"
 
+#include <type_traits>
+
 namespace {
 
 using jg::BlockOf;
@@ -60,9 +62,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int D = 64;
-constexpr int BR = 128;           // resident rows per workgroup (4 blocks of 32)
 constexpr int BT = 64;            // streamed rows per tile
-constexpr int THREADS = 512;
 constexpr int ROWB = D * 2;       // bytes per row of a tile in LDS (no padding)
 constexpr int NAT = BT * ROWB;    // 8192: one 64 x 64 bf16 tile
 constexpr float LOG2E = 1.4426950408889634f;
@@ -147,44 +147,55 @@ struct BwdArgs {
 };
 
 // ------------------------------------------------------------------ dQ kernel
-constexpr int NBUF = 4;                     // tiles in flight per half: read back, current, read ahead, landing
-constexpr int DQ_BUF = 2 * NAT;             // K tile, V tile
-constexpr int DQ_HALF = NBUF * DQ_BUF;
-constexpr int DQ_LDS = 2 * DQ_HALF;         // 131072 (and at least 4 x 32 x 64 floats for the hand-over)
+constexpr int NBUF = 4;                     // tiles of a half in LDS: read back, current, read ahead, landing
+// QB: query blocks per workgroup, 4 or 2. A tile holds 16 keys a query block: every wavefront moves 16 rows of it.
+template <int QB>
+struct DqPlan {
+  static constexpr int THREADS = 64 * 2 * QB;
+  static constexpr int ROWS = 32 * QB;        // queries
+  static constexpr int TILE = 16 * QB;        // keys
+  static constexpr int BLOCKS = TILE / 32;    // blocks of the pipeline in a tile
+  static constexpr int BYTES = TILE * ROWB;
+  static constexpr int BUF = 2 * BYTES;       // K tile, V tile
+  static constexpr int HALF = NBUF * BUF;
+  static constexpr int LDS = 2 * HALF;        // 131072 or 65536
+  static_assert(LDS >= QB * 32 * 64 * 4, "the hand-over of the partial dQ reuses the tile buffers");
+};
 
 // Scheduling classes of __builtin_amdgcn_sched_group_barrier
 #define JG_GROUP_VALU 0x002
 #define JG_GROUP_MFMA 0x008
 #define JG_GROUP_DS_READ 0x100
 
-template <bool RAGGED>
-__global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks, BwdArgs p) {
+template <bool RAGGED, int QB>
+__global__ __launch_bounds__(DqPlan<QB>::THREADS, QB == 2 ? 2 : 1) void attn_bwd_dq_kernel(ChunkTable chunks, BwdArgs p) {
+  constexpr int DQ_BT = DqPlan<QB>::TILE, DQ_NAT = DqPlan<QB>::BYTES, DQ_BUF = DqPlan<QB>::BUF, BLOCKS = DqPlan<QB>::BLOCKS;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kg = lane >> 5;
-  const int qb = wave & 3, ks = wave >> 2;
+  const int qb = wave % QB, ks = wave / QB;
   const BlockOf where = block_of();
   const long long b = where.bh;
-  const int q0 = where.blk * BR + qb * 32;
+  const int q0 = where.blk * DqPlan<QB>::ROWS + qb * 32;
   // every chunk is cut in two key halves (one per wavefront group); a half's tiles of all chunks
   // form one stream of ntiles tiles
-  const int tiles_per_chunk = (p.sk + 2 * BT - 1) / (2 * BT);
+  const int tiles_per_chunk = (p.sk + 2 * DQ_BT - 1) / (2 * DQ_BT);
   const int ntiles = tiles_per_chunk * p.nchunks;
   const float c2 = p.scale * LOG2E;
   const bool q_live = !RAGGED || q0 + ln < p.sq;
   const long long qi = b * p.sq + (q_live ? q0 + ln : p.sq - 1);
 
-  unsigned char* lds = smem + ks * DQ_HALF;
+  unsigned char* lds = smem + ks * DqPlan<QB>::HALF;
   // this wavefront moves rows 16 qb .. 16 qb + 15 of the K tile and of the V tile of its half
   const int ks_u = __builtin_amdgcn_readfirstlane(ks), qb_u = __builtin_amdgcn_readfirstlane(qb);
   const long long chunk_off = 2 * (b * p.sk * (long long)D);  // bytes into a chunk
-  const int row_first = ks_u * tiles_per_chunk * BT + 16 * qb_u;
+  const int row_first = ks_u * tiles_per_chunk * DQ_BT + 16 * qb_u;
   int ld_chunk = 0, ld_tile = 0;  // the load cursor: tiles are requested in stream order
   const char* kdma = chunk_entry(0, 0) + chunk_off;
   const char* vdma = chunk_entry(1, 0) + chunk_off;
   const uint32_t dma_off = dma_lane_offset(lane);
-  const uint32_t lds_dma = lds_address(smem) + (uint32_t)(ks_u * DQ_HALF + 16 * qb_u * ROWB);
+  const uint32_t lds_dma = lds_address(smem) + (uint32_t)(ks_u * DqPlan<QB>::HALF + 16 * qb_u * ROWB);
   const int tr_off[2] = {tr_lane_offset(lane, 0), tr_lane_offset(lane, 1)};
   // row fragments: row ln of a 32-row block, chunk 2 c + kg
   int row_off[4];
@@ -192,21 +203,21 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
   for (int c = 0; c < 4; ++c) row_off[c] = ln * ROWB + (((2 * c + kg) ^ (ln & 7)) << 4);
 
   // K and V of tile t straight into its buffer (free since the barrier that ended the tile before)
-  auto issue_loads = [&](int t) {  // called with t = 0, 1, 2, ... in turn
-    const uint32_t dst = lds_dma + (uint32_t)((t & (NBUF - 1)) * DQ_BUF);
-    const int row = row_first + ld_tile * BT;
+  auto issue_loads = [&](int slot) {  // called with slot = 0, 1, 2, 3, 0, ... in turn
+    const uint32_t dst = lds_dma + (uint32_t)(slot * DQ_BUF);
+    const int row = row_first + ld_tile * DQ_BT;
     if (RAGGED) {
       const uint32_t o0 = dma_clamped_offset(lane, row, p.sk), o1 = dma_clamped_offset(lane, row + 8, p.sk);
       dma_1k(kdma, o0, dst);
       dma_1k(kdma, o1, dst + 8 * ROWB);
-      dma_1k(vdma, o0, dst + NAT);
-      dma_1k(vdma, o1, dst + NAT + 8 * ROWB);
+      dma_1k(vdma, o0, dst + DQ_NAT);
+      dma_1k(vdma, o1, dst + DQ_NAT + 8 * ROWB);
     } else {
       const long long off = (long long)row * ROWB;
       dma_1k(kdma + off, dma_off, dst);
       dma_1k(kdma + off + 8 * ROWB, dma_off, dst + 8 * ROWB);
-      dma_1k(vdma + off, dma_off, dst + NAT);
-      dma_1k(vdma + off + 8 * ROWB, dma_off, dst + NAT + 8 * ROWB);
+      dma_1k(vdma + off, dma_off, dst + DQ_NAT);
+      dma_1k(vdma + off + 8 * ROWB, dma_off, dst + DQ_NAT + 8 * ROWB);
     }
     if (++ld_tile == tiles_per_chunk && ld_chunk + 1 < p.nchunks) {
       ld_tile = 0;
@@ -214,9 +225,6 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
       kdma = chunk_entry(0, ld_chunk) + chunk_off;
       vdma = chunk_entry(1, ld_chunk) + chunk_off;
     }
-  };
-  auto tiles_landed = [&]() {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's transfers have landed
   };
 
   // the first tiles are on their way while the wavefront fetches its own rows
@@ -267,7 +275,7 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lds_frag(kn + sb * 32 * ROWB + row_off[c]), qf[c], s, 0, 0, 0);
-      dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lds_frag(kn + NAT + sb * 32 * ROWB + row_off[c]), dof[c], dp, 0, 0, 0);
+      dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lds_frag(kn + DQ_NAT + sb * 32 * ROWB + row_off[c]), dof[c], dp, 0, 0, 0);
     }
   };
   auto ds_frag = [&](int t) {
@@ -287,7 +295,7 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
         dq[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(kn, tr_off[nb], sb * 32 + 16 * t), ds_prev[t], dq[nb], 0, 0, 0);
   };
   // one step of the pipeline: A of (k_next, sb_next), B of the current block, C of (k_prev, sb_prev)
-  int keys_left = p.sk - ks_u * tiles_per_chunk * BT, tile_at = 0;  // RAGGED: keys from the current block's first one on
+  int keys_left = p.sk - ks_u * tiles_per_chunk * DQ_BT, tile_at = 0;  // RAGGED: keys from the current block's first one on
   auto step = [&](const unsigned char* k_next, int sb_next, const unsigned char* k_prev, int sb_prev, bool ahead) {
     if (RAGGED) {
       if (keys_left < 32) {
@@ -296,9 +304,9 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
           if (8 * (i >> 2) + 4 * kg + (i & 3) >= keys_left) s_cur[i] = -INFINITY;
       }
       keys_left -= 32;
-      if (++tile_at == 2 * tiles_per_chunk) {  // the next block opens the next chunk
+      if (++tile_at == BLOCKS * tiles_per_chunk) {  // the next block opens the next chunk
         tile_at = 0;
-        keys_left += tiles_per_chunk * BT;
+        keys_left += tiles_per_chunk * DQ_BT;
       }
     }
     f32x16 s_n, dp_n;
@@ -322,7 +330,7 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
     ds_prev[1] = ds_now[1];
   };
 
-  tiles_landed();
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's transfers have landed
   __syncthreads();
   scores(lds, 0, s_cur, dp_cur);
 #pragma unroll
@@ -330,25 +338,34 @@ __global__ __launch_bounds__(THREADS) void attn_bwd_dq_kernel(ChunkTable chunks,
     ds_prev[0][i] = (__bf16)0.0f;  // block -1 adds nothing (times the finite K of block 0)
     ds_prev[1][i] = (__bf16)0.0f;
   }
-  const unsigned char* k_back = lds;  // tile of the block before the current one
-  int sb_back = 0;
-  for (int t = 0; t + 1 < ntiles; ++t) {
-    if (t + 2 < ntiles) issue_loads(t + 2);
-    const unsigned char* kn = lds + (t & (NBUF - 1)) * DQ_BUF;
-    const unsigned char* kn1 = lds + ((t + 1) & (NBUF - 1)) * DQ_BUF;
-    step(kn, 1, k_back, sb_back, true);
-    step(kn1, 0, kn, 0, true);
-    k_back = kn;
-    sb_back = 1;
-    tiles_landed();
+  // Four tiles a round: a tile's buffer is then a constant offset of the LDS reads (8 heads x 4096 queries x 4 chunks 212 -> 203 us).
+  auto tile = [&](int slot) { return lds + slot * DQ_BUF; };
+  // all blocks of tile t, in buffer `slot`: each with the scores of the block behind it and the block before it added
+  auto advance = [&](int t, int slot, bool last) __attribute__((always_inline)) {
+    const unsigned char* const kn = tile(slot);
+    const unsigned char* const back = t == 0 ? lds : tile((slot + 3) % NBUF);
+    if (BLOCKS == 2) {
+      step(kn, 1, back, t == 0 ? 0 : 1, true);
+      step(tile((slot + 1) % NBUF), 0, kn, 0, !last);
+    } else {
+      step(tile((slot + 1) % NBUF), 0, back, 0, !last);
+    }
+  };
+  auto advance_more = [&](int t, int slot) __attribute__((always_inline)) {
+    if (t + 2 < ntiles) issue_loads((slot + 2) % NBUF);
+    advance(t, slot, false);
+    __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
+  };
+  int t = 0;
+  for (; t + NBUF < ntiles; t += NBUF) {
+#pragma unroll
+    for (int i = 0; i < NBUF; ++i) advance_more(t + i, i);
   }
-  {
-    const unsigned char* kn = lds + ((ntiles - 1) & (NBUF - 1)) * DQ_BUF;
-    step(kn, 1, k_back, sb_back, true);
-    step(kn, 0, kn, 0, false);
-    add_to_dq(kn, 1);
-  }
+#pragma unroll 1
+  for (; t + 1 < ntiles; ++t) advance_more(t, t % NBUF);
+  advance(t, t % NBUF, true);
+  add_to_dq(tile(t % NBUF), BLOCKS - 1);
   __syncthreads();  // the hand-over below reuses the tile buffers
 
   // combine the two key halves, then write dQ (lane = query, 4 consecutive d per store)
@@ -603,18 +620,30 @@ int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
     auto reserve = [](const void* f, int bytes) {
       return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
     };
-    if (!reserve(reinterpret_cast<const void*>(&attn_bwd_dq_kernel<false>), DQ_LDS) ||
-        !reserve(reinterpret_cast<const void*>(&attn_bwd_dq_kernel<true>), DQ_LDS) ||
+    if (!reserve(reinterpret_cast<const void*>(&attn_bwd_dq_kernel<false, 4>), DqPlan<4>::LDS) ||
+        !reserve(reinterpret_cast<const void*>(&attn_bwd_dq_kernel<true, 4>), DqPlan<4>::LDS) ||
+        !reserve(reinterpret_cast<const void*>(&attn_bwd_dq_kernel<false, 2>), DqPlan<2>::LDS) ||
+        !reserve(reinterpret_cast<const void*>(&attn_bwd_dq_kernel<true, 2>), DqPlan<2>::LDS) ||
         !reserve(reinterpret_cast<const void*>(&attn_bwd_dkv_kernel<false>), DKV_LDS) ||
         !reserve(reinterpret_cast<const void*>(&attn_bwd_dkv_kernel<true>), DKV_LDS))
       JG_FAIL(JG_ERR_LAUNCH, "jg_attn_bwd: cannot reserve LDS");
     attr_set = true;
   }
-  const bool ragged = sq % BR != 0 || sk % BR != 0 || sk % DKV_ROWS != 0;
-  const dim3 dq_grid((unsigned)cdiv(sq, BR), (unsigned)batch, 1);
+  const bool ragged = sq % (2 * BT) != 0 || sk % (2 * BT) != 0;
+  auto launch_dq = [&](auto qb_c) {
+    constexpr int QB = decltype(qb_c)::value;
+    typedef DqPlan<QB> Plan;
+    const dim3 grid((unsigned)cdiv(sq, Plan::ROWS), (unsigned)batch, 1);
+    if (ragged) attn_bwd_dq_kernel<true, QB><<<grid, Plan::THREADS, Plan::LDS, s>>>(tab, a);
+    else attn_bwd_dq_kernel<false, QB><<<grid, Plan::THREADS, Plan::LDS, s>>>(tab, a);
+  };
   const dim3 dkv_grid((unsigned)cdiv(sk, DKV_ROWS), (unsigned)batch, (unsigned)nchunks);
-  if (ragged) attn_bwd_dq_kernel<true><<<dq_grid, THREADS, DQ_LDS, s>>>(tab, a);
-  else attn_bwd_dq_kernel<false><<<dq_grid, THREADS, DQ_LDS, s>>>(tab, a);
+  // Where workgroups of 128 queries would leave half of the compute units without one, those of 64 queries (128 : 64, us): 8 heads x
+  // 2048 queries x 4 chunks 94 : 81, 3 x 4000 x 8 321 : 285, 18 x 700 x 3 32 : 26, 10 x 284 x 3 19 : 13. Elsewhere twice the tile
+  // traffic and a barrier for half the keys cost more than the waves' independence gives: 8 x 4096 x 4 203 : 223, 32 x 1024 x 1
+  // 18.0 : 18.9, 24 x 1000 x 2 30.8 : 32.1.
+  if (2 * batch * cdiv(sq, DqPlan<4>::ROWS) <= cu_count()) launch_dq(std::integral_constant<int, 2>{});
+  else launch_dq(std::integral_constant<int, 4>{});
   JG_CHECK_LAUNCH("jg_attn_bwd(dq)");
   if (ragged) attn_bwd_dkv_kernel<true><<<dkv_grid, DKV_THREADS, DKV_LDS, s>>>(tab, a);
   else attn_bwd_dkv_kernel<false><<<dkv_grid, DKV_THREADS, DKV_LDS, s>>>(tab, a);

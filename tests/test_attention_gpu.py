@@ -354,6 +354,24 @@ def test_backward_over_resident_chunks_in_one_pass(b, h, n, nk, P, dev):
     assert torch.equal(dq2, dq) and all(torch.equal(a, c) for a, c in zip(dks2, dks))
 
 
+@pytest.mark.parametrize("heads", [2, 150], ids=["64-query workgroups", "128-query workgroups"])
+@pytest.mark.parametrize("n,nk,P", [(64, 128, 1), (65, 129, 1), (128, 192, 1), (127, 257, 1), (33, 320, 1), (96, 383, 1), (130, 448, 1), (64, 640, 1), (100, 1100, 1),
+                                    (64, 128, 2), (70, 190, 3), (128, 256, 5)], ids=str)
+def test_query_gradient_at_the_ends_of_its_key_tiles(heads, n, nk, P, dev):
+    """One to eighteen tiles of a key half (four a round, then one by one), chunks that end inside a tile, both workgroup sizes. dS is rounded to bf16,
+    half of 2^-8, and so is the result; twice that leaves room for the exponential and the sums."""
+    torch.manual_seed(n + nk)
+    d, scale = 64, 0.125
+    q, dout = (torch.randn(1, heads, n, d, device=dev).bfloat16() for _ in range(2))
+    ks, vs = ([torch.randn(1, heads, nk, d, device=dev).bfloat16() for _ in range(P)] for _ in range(2))
+    out, lse = ja.ring_forward(q, ks, vs, scale, rank=0)
+    dq, _, _ = ja.ring_backward(dout, q, out, lse, ks, vs, scale)
+    Q, K, V, dO, O, L = (t[0].double().cpu() for t in (q, torch.cat(ks, 2), torch.cat(vs, 2), dout, out, lse))
+    dS = torch.exp(Q @ K.mT * scale - L[..., None]) * (dO @ V.mT - (dO * O).sum(-1, keepdim=True)) * scale
+    off = (dq[0].double().cpu() - dS @ K).abs() - 2.0**-8 * (dS.abs() @ K.abs() + (dS @ K).abs())
+    assert off.max() <= 0, off.max()
+
+
 def test_backward_over_chunks_declines_what_it_does_not_cover(dev):
     q = torch.randn(1, 1, 128, 64, device=dev)
     k = [torch.randn(1, 1, 128, 64, device=dev)]
