@@ -14,24 +14,29 @@
 //                  CUs, more wavefronts share the rows of one (see split_of on the host side).
 //
 // Forward + backward of a ring, before (lengths and head size padded on the host, one launch and one merge per
-// chunk) and now: 4 heads x 128 x 2 chunks of 128 keys, head size 32: 402 -> 48 us (host time); 12 heads x 869 x 869,
+// chunk) and in one launch each: 4 heads x 128 x 2 chunks of 128 keys, head size 32: 402 -> 48 us (host time); 12 heads x 869 x 869,
 // head size 96, fp16: 528 -> 99 us; 16 heads x 2424 x 2424, head size 32, fp16: 568 -> 225 us.
 //
 //   forward / dQ   lane = query. S^T = K Q^T (A = K rows from LDS, B = Q rows kept in
 //                  registers), so the running max / sum, lse and delta of a query are
 //                  scalars of the two lanes that share it. P^T (or dS^T) leaves the
 //                  accumulator already in B-fragment position for O^T += V^T P^T
-//                  (dQ^T += K^T dS^T): the A operand is a transposed copy of the tile in
-//                  LDS whose 32 columns are stored in the order the accumulator holds its
-//                  rows.
+//                  (dQ^T += K^T dS^T): the A operand comes from the same tile by LDS transpose
+//                  reads, its 16 rows in the order the accumulator holds them.
 //   dK / dV        lane = key. S = Q K^T and dP = dO V^T with K, V rows in registers;
 //                  lse and delta of the tile's queries are read from LDS per accumulator
-//                  row; dV^T += dO^T P and dK^T += Q^T dS use transposed copies of the dO
+//                  row; dV^T += dO^T P and dK^T += Q^T dS by transpose reads of the dO
 //                  and Q tiles.
+//
+// A transposed copy of the tile beside it, fetched and written a second time, had these kernels at (copy : transpose reads, with the loads
+// above; forward / dQ / dK and dV, us) 6 heads x 4050 x 4 chunks, head size 80 460 / 559 / 931 : 339 / 357 / 366; 24 x 1000 x 2, 128
+// 65 / 83 / 125 : 60 / 65 / 110; 24 x 739 x 5, 32 54 / 62 / 52 : 48 / 46 / 31; 8 x 4096 x 2, fp16 64 193 / 240 / 195 : 186 / 173 / 161. What is
+// left is one chain per wavefront, scores, exponentials, products, with two wavefronts a SIMD to fill its gaps.
 //
 // Reference behaviour restated here:
 //   jigsaw/modules/attention/_functional/cores/math.py:69-78   (forward)
 //   jigsaw/modules/attention/_functional/cores/math.py:125-149 (backward)
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_chunks.h"
@@ -53,6 +58,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef short i16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int WAVES = 4, GROUP = WAVES * 64;  // wavefronts and threads of a group
 constexpr int BQ = 32 * WAVES;  // rows (queries or keys) of a workgroup, 32 per wavefront of a group
@@ -63,90 +69,47 @@ constexpr float NO_SCORE = -1.0e30f;  // running maximum before the first key: f
 template <int D>
 struct Geo {
   static constexpr int C16 = D / 16, NB = D / 32;
-  static constexpr int RP = D * 2 + 16;   // bytes per row of a row-major tile (32 rows of D): an odd number of 16-byte units
-  static constexpr int TP = BT * 2 + 16;  // bytes per row of a transposed tile (D rows of 32)
-  static constexpr int ROWMAJ = BT * RP, TRANS = D * TP;
+  static constexpr int RP = D * 2;  // bytes per row of a tile (32 rows of D)
+  static constexpr int TILE = BT * RP;
+  // Row r has its 16-byte pieces XOR-ed with swizzle(r). The 16 rows a row fragment's read takes at a time then meet all banks once, and so do
+  // the 64 bytes of 4 rows of a transposed fragment. (Rows 16 bytes apart instead: two to a bank there; dQ of 8 heads x 4096 x 2 chunks at head
+  // size 96 270 : 240 us, fp16 64 211 : 188.)
+  __device__ static __forceinline__ int swizzle(int r) { return ((r >> 2) & 3) | (D == 64 ? ((r >> 1) & 1) << 2 : (D == 128 ? (r & 3) << 2 : 0)); }
+  static constexpr int RV = D == 64 ? 4 : (D == 128 ? 8 : 2), TV = RV / 2;  // pieces, and blocks of 32 columns, whose swizzles differ
   static constexpr int CHUNKS = BT * D / 8;  // 16-byte pieces of a tile
   static constexpr int PER = (CHUNKS + GROUP - 1) / GROUP;
 };
 
-// Column of a transposed tile that holds tile row x: inside a group of 16 rows the order is the
-// one in which an MFMA accumulator lane holds its rows, so that probabilities need no shuffle on
-// their way from accumulator to B operand: 16*(x/16) + ((x%8)/4)*8 + ((x%16)/8)*4 + x%4.
-
 template <int D>
 struct TileRegs {
   u32x4 v[Geo<D>::PER];
+  int rows;
 };
 
-// 32 rows of a row-major matrix of row length d <= D to registers; rows from `rows` on and columns from d on are
-// zero. tid: thread of the group.
+// 32 rows of a row-major matrix of row length d <= D to registers; rows from `rows` on and columns from d on become zero on their way to LDS.
+// They are read from the last row and piece there is: a load under a condition is waited for where the paths meet, on the spot (24 heads x
+// 739 x 5 chunks, head size 32: forward 63 -> 48 us, dQ 54 -> 46). tid: thread of the group; at least one row lies before `rows`.
 template <int D>
 __device__ __forceinline__ void tile_fetch(TileRegs<D>& r, const uint16_t* src, int tid, int rows, int d) {
-  if (rows >= BT && d == D) {  // wave-uniform
-#pragma unroll
-    for (int i = 0; i < Geo<D>::PER; ++i) {
-      const int c = tid + i * GROUP;
-      if (c < Geo<D>::CHUNKS) r.v[i] = *reinterpret_cast<const u32x4*>(src + c * 8);  // rows are contiguous: chunk c = 8 elements at c*8
-    }
-    return;
-  }
+  r.rows = rows;
 #pragma unroll
   for (int i = 0; i < Geo<D>::PER; ++i) {
-    const int c = tid + i * GROUP;
-    const int row = c / (D / 8), col = (c % (D / 8)) * 8;
-    r.v[i] = u32x4{0u, 0u, 0u, 0u};
-    if (c < Geo<D>::CHUNKS && row < rows && col < d) r.v[i] = *reinterpret_cast<const u32x4*>(src + row * d + col);
+    const int c = min(tid + i * GROUP, Geo<D>::CHUNKS - 1);
+    r.v[i] = *reinterpret_cast<const u32x4*>(src + min(c / (D / 8), rows - 1) * d + min(c % (D / 8) * 8, d - 8));
   }
 }
 template <int D>
-__device__ __forceinline__ void tile_store_rows(const TileRegs<D>& r, unsigned char* dst, int tid) {
+__device__ __forceinline__ void tile_store(const TileRegs<D>& r, unsigned char* dst, int tid, int d) {
 #pragma unroll
   for (int i = 0; i < Geo<D>::PER; ++i) {
     const int c = tid + i * GROUP;
     if (c < Geo<D>::CHUNKS) {
-      const int row = c / (D / 8), col8 = c % (D / 8);
-      *reinterpret_cast<u32x4*>(dst + row * Geo<D>::RP + col8 * 16) = r.v[i];
-    }
-  }
-}
-// Transposed staging: a thread takes 8 rows x 2 columns of the tile (8 dwords) and writes, for each
-// of its two columns, the 8 values as two 8-byte pieces of the transposed tile's row.
-template <int D>
-struct TransRegs {
-  uint32_t w[8];
-};
-template <int D>
-__device__ __forceinline__ void trans_fetch(TransRegs<D>& r, const uint16_t* src, int tid, int rows, int d) {
-  if (tid < 4 * (D / 2)) {
-    const int g8 = tid / (D / 2), cp = tid % (D / 2);
-    if (rows >= BT && d == D) {  // wave-uniform
+      const int row = c / (D / 8), piece = c % (D / 8);
+      const bool there = row < r.rows && piece * 8 < d;
+      u32x4 v;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) r.w[i] = *reinterpret_cast<const uint32_t*>(src + (g8 * 8 + i) * D + 2 * cp);
-      return;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      r.w[i] = (g8 * 8 + i < rows && 2 * cp < d) ? *reinterpret_cast<const uint32_t*>(src + (g8 * 8 + i) * d + 2 * cp) : 0u;
-  }
-}
-template <int D>
-__device__ __forceinline__ void trans_store(const TransRegs<D>& r, unsigned char* dst, int tid) {
-  if (tid < 4 * (D / 2)) {
-    const int g8 = tid / (D / 2), cp = tid % (D / 2);
-    // rows 8*g8 .. 8*g8+7 of the tile: the first four land at the place of row 8*g8, the last four 8 places on
-    const int pos_lo = (g8 >> 1) * 16 + (g8 & 1) * 4, pos_hi = pos_lo + 8;
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const uint32_t sel = e ? 0x07060302u : 0x05040100u;
-      u32x2 lo, hi;
-      lo.x = __builtin_amdgcn_perm(r.w[1], r.w[0], sel);
-      lo.y = __builtin_amdgcn_perm(r.w[3], r.w[2], sel);
-      hi.x = __builtin_amdgcn_perm(r.w[5], r.w[4], sel);
-      hi.y = __builtin_amdgcn_perm(r.w[7], r.w[6], sel);
-      unsigned char* row = dst + (2 * cp + e) * Geo<D>::TP;
-      *reinterpret_cast<u32x2*>(row + pos_lo * 2) = lo;
-      *reinterpret_cast<u32x2*>(row + pos_hi * 2) = hi;
+      for (int e = 0; e < 4; ++e) v[e] = there ? r.v[i][e] : 0u;
+      *reinterpret_cast<u32x4*>(dst + row * Geo<D>::RP + ((piece ^ Geo<D>::swizzle(row)) << 4)) = v;
     }
   }
 }
@@ -196,6 +159,38 @@ template <bool F16>
 __device__ __forceinline__ typename Half<F16>::x8 frag(const unsigned char* at) {
   return __builtin_bit_cast(typename Half<F16>::x8, *reinterpret_cast<const u32x4*>(at));
 }
+// Where a lane finds its parts of a tile: fragments of row ln (columns 16 c + 8 kg + 0..7), and transposed ones by LDS transpose reads (within
+// 16 lanes, lane i receives element i % 4 of the 8 bytes that lanes i / 4 + 4 j point at, j = 0..3): lane (ln, kg) gets column ln of
+// block nb and, of 16 rows, rows 4 kg + 0..3 and 8 + 4 kg + 0..3, the order in which an accumulator lane holds its rows.
+template <int D, bool F16>
+struct TileView {
+  typedef Geo<D> G;
+  typedef typename Half<F16>::x8 X8;
+  int row[G::RV], lo[G::TV], hi[G::TV];
+  __device__ __forceinline__ explicit TileView(int lane) {
+    const int ln = lane & 31, kg = lane >> 5, p = lane & 15, r = 4 * kg + (p >> 2);
+#pragma unroll
+    for (int c = 0; c < G::RV; ++c) row[c] = ln * G::RP + (((2 * c + kg) ^ G::swizzle(ln)) << 4);
+#pragma unroll
+    for (int v = 0; v < G::TV; ++v) {
+      const int piece = 4 * v + ((lane >> 4) & 1) * 2 + ((p >> 1) & 1);
+      lo[v] = r * G::RP + ((piece ^ G::swizzle(r)) << 4) + 8 * (p & 1);
+      hi[v] = (r + 8) * G::RP + ((piece ^ G::swizzle(r + 8)) << 4) + 8 * (p & 1);
+    }
+  }
+  __device__ __forceinline__ X8 rows(const unsigned char* tile, int c) const { return frag<F16>(tile + row[c % G::RV] + c / G::RV * 64); }
+  __device__ __forceinline__ X8 trans(const unsigned char* tile, int nb, int half) const {  // rows 16 half + ...
+    typedef __attribute__((address_space(3))) i16x4* tr_ptr;
+    const unsigned char* const at = tile + nb / G::TV * 64 + half * 16 * G::RP;
+    const i16x4 l = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at + lo[nb % G::TV])), h = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at + hi[nb % G::TV]));
+    u32x4 w;
+    w.x = __builtin_bit_cast(u32x2, l).x;
+    w.y = __builtin_bit_cast(u32x2, l).y;
+    w.z = __builtin_bit_cast(u32x2, h).x;
+    w.w = __builtin_bit_cast(u32x2, h).y;
+    return __builtin_bit_cast(X8, w);
+  }
+};
 template <bool F16>
 __device__ __forceinline__ typename Half<F16>::x8 pack8(const float* v) {
   u32x4 r;
@@ -293,7 +288,7 @@ template <int D, bool F16, int KS, bool EXACT>
 __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, Args p) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
-  constexpr int BUF = G::ROWMAJ + G::TRANS;  // K rows, then V^T
+  constexpr int BUF = 2 * G::TILE;  // K tile, V tile
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x % GROUP, ks = threadIdx.x / GROUP;
   const int lane = tid & 63, wave = tid >> 6;
@@ -306,6 +301,7 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
   const long long chunk_off = bh * p.sk * p.d;
   const float c2 = p.scale * LOG2E;
   unsigned char* lds = smem + ks * 2 * BUF;
+  const TileView<D, F16> view(lane);
 
   X8 qf[G::C16];
 #pragma unroll
@@ -322,8 +318,7 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
     const bool exact = EXACT && pass == 1;
     const int lo = exact ? p.exact_from : 0, hi = EXACT && !exact ? p.exact_from : p.sk;
     if (EXACT && lo == hi) continue;
-    TileRegs<D> rk;
-    TransRegs<D> rv;
+    TileRegs<D> rk, rv;
     Stream<KS> load(lo, hi, ks), soft(lo, hi, ks);
     const int ntiles = load.steps * p.nchunks;
     auto fetch = [&]() {
@@ -331,12 +326,12 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
       const uint16_t* vb = reinterpret_cast<const uint16_t*>(chunk_entry(1, load.chunk)) + chunk_off;
       const long long at = (long long)load.first_row() * p.d;
       tile_fetch<D>(rk, kb + at, tid, load.rows_left(), p.d);
-      trans_fetch<D>(rv, vb + at, tid, load.rows_left(), p.d);
+      tile_fetch<D>(rv, vb + at, tid, load.rows_left(), p.d);
       load.next();
     };
     auto store = [&](int buf) {
-      tile_store_rows<D>(rk, lds + buf * BUF, tid);
-      trans_store<D>(rv, lds + buf * BUF + G::ROWMAJ, tid);
+      tile_store<D>(rk, lds + buf * BUF, tid, p.d);
+      tile_store<D>(rv, lds + buf * BUF + G::TILE, tid, p.d);
     };
     fetch();
     store(0);
@@ -348,13 +343,13 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
     __syncthreads();
     for (int t = 0; t < ntiles; ++t) {
       const unsigned char* kt = lds + (t & 1) * BUF;
-      const unsigned char* vt = kt + G::ROWMAJ;
+      const unsigned char* vt = kt + G::TILE;
       if (t + 1 < ntiles) fetch();
       // S^T: lane = query ln, register i = key 8*(i/4) + 4*kg + i%4 of the tile
       f32x16 s = zero16();
 #pragma unroll
       for (int c = 0; c < G::C16; ++c)
-        s = Half<F16>::mma(frag<F16>(kt + ln * G::RP + (16 * c + 8 * kg) * 2), qf[c], s);
+        s = Half<F16>::mma(view.rows(kt, c), qf[c], s);
       if (soft.rows_left() < BT) {  // wave-uniform
 #pragma unroll
         for (int i = 0; i < 16; ++i)
@@ -386,16 +381,15 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
       l += sum;
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        const unsigned char* at = vt + ln * G::TP + (16 * ks + 8 * kg) * 2;
         if (exact) {
           bf16x8 part[3];
           parts8<true>(pr + 8 * ks, part);
 #pragma unroll
-          for (int nb = 0; nb < G::NB; ++nb) o[nb] = mma_exact<F16>(frag<F16>(at + nb * 32 * G::TP), part, o[nb]);
+          for (int nb = 0; nb < G::NB; ++nb) o[nb] = mma_exact<F16>(view.trans(vt, nb, ks), part, o[nb]);
         } else {
           const X8 pf = pack8<F16>(pr + 8 * ks);
 #pragma unroll
-          for (int nb = 0; nb < G::NB; ++nb) o[nb] = Half<F16>::mma(frag<F16>(at + nb * 32 * G::TP), pf, o[nb]);
+          for (int nb = 0; nb < G::NB; ++nb) o[nb] = Half<F16>::mma(view.trans(vt, nb, ks), pf, o[nb]);
         }
       }
       if (t + 1 < ntiles) store((t + 1) & 1);
@@ -406,8 +400,7 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
   l += __shfl_xor(l, 32, 64);
   if constexpr (KS > 1) {
     // the groups hand over to the one below them, halving their number each time
-    constexpr int XO = (16 * G::NB + 2) * 64;  // floats of a wavefront
-    static_assert(KS / 2 * WAVES * XO * 4 <= KS * 2 * BUF, "the hand-over reuses the stages");
+    constexpr int XO = (16 * G::NB + 2) * 64;  // floats of a wavefront (in the stages' place, see launch_fwd)
     float* xo = reinterpret_cast<float*>(smem) + ((ks % (KS / 2)) * WAVES + wave) * XO + lane;
 #pragma unroll
     for (int half = KS / 2; half >= 1; half >>= 1) {
@@ -479,7 +472,7 @@ template <int D, bool F16, int KS, bool EXACT>
 __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Args p) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
-  constexpr int BUF = 2 * G::ROWMAJ + G::TRANS;  // K rows, V rows, K^T
+  constexpr int BUF = 2 * G::TILE;  // K tile, V tile
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x % GROUP, ks = threadIdx.x / GROUP;
   const int lane = tid & 63, wave = tid >> 6;
@@ -492,6 +485,7 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
   const long long chunk_off = bh * p.sk * p.d;
   const float c2 = p.scale * LOG2E;
   unsigned char* lds = smem + ks * 2 * BUF;
+  const TileView<D, F16> view(lane);
 
   X8 qf[G::C16], dof[G::C16];
   float dl = 0.0f;
@@ -513,7 +507,6 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
   for (int nb = 0; nb < G::NB; ++nb) dq[nb] = zero16();
 
   TileRegs<D> rk, rv;
-  TransRegs<D> rkt;
   Stream<KS> load(0, p.sk, ks), soft(0, p.sk, ks);
   const int ntiles = load.steps * p.nchunks;
   auto fetch = [&]() {
@@ -522,14 +515,12 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
     const uint16_t* vb = reinterpret_cast<const uint16_t*>(chunk_entry(1, load.chunk)) + at;
     tile_fetch<D>(rk, kb, tid, load.rows_left(), p.d);
     tile_fetch<D>(rv, vb, tid, load.rows_left(), p.d);
-    trans_fetch<D>(rkt, kb, tid, load.rows_left(), p.d);
     load.next();
   };
   auto store = [&](int buf) {
     unsigned char* at = lds + buf * BUF;
-    tile_store_rows<D>(rk, at, tid);
-    tile_store_rows<D>(rv, at + G::ROWMAJ, tid);
-    trans_store<D>(rkt, at + 2 * G::ROWMAJ, tid);
+    tile_store<D>(rk, at, tid, p.d);
+    tile_store<D>(rv, at + G::TILE, tid, p.d);
   };
   fetch();
   store(0);
@@ -539,14 +530,13 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
   __syncthreads();
   for (int t = 0; t < ntiles; ++t) {
     const unsigned char* kt = lds + (t & 1) * BUF;
-    const unsigned char* vt = kt + G::ROWMAJ;
-    const unsigned char* ktt = kt + 2 * G::ROWMAJ;
+    const unsigned char* vt = kt + G::TILE;
     if (t + 1 < ntiles) fetch();
     f32x16 s = zero16(), dp = zero16();
 #pragma unroll
     for (int c = 0; c < G::C16; ++c) {
-      s = Half<F16>::mma(frag<F16>(kt + ln * G::RP + (16 * c + 8 * kg) * 2), qf[c], s);
-      dp = Half<F16>::mma(frag<F16>(vt + ln * G::RP + (16 * c + 8 * kg) * 2), dof[c], dp);
+      s = Half<F16>::mma(view.rows(kt, c), qf[c], s);
+      dp = Half<F16>::mma(view.rows(vt, c), dof[c], dp);
     }
     if (soft.rows_left() < BT) {  // wave-uniform
 #pragma unroll
@@ -559,23 +549,22 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
     for (int i = 0; i < 16; ++i) ds[i] = __builtin_amdgcn_exp2f(s[i] * c2 - lse2) * (dp[i] - delta);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      const unsigned char* at = ktt + ln * G::TP + (16 * ks + 8 * kg) * 2;
       if constexpr (EXACT) {
         bf16x8 part[3];
         parts8<false>(ds + 8 * ks, part);
 #pragma unroll
-        for (int nb = 0; nb < G::NB; ++nb) dq[nb] = mma_exact<F16>(frag<F16>(at + nb * 32 * G::TP), part, dq[nb]);
+        for (int nb = 0; nb < G::NB; ++nb) dq[nb] = mma_exact<F16>(view.trans(kt, nb, ks), part, dq[nb]);
       } else {
         const X8 dsf = pack8<F16>(ds + 8 * ks);
 #pragma unroll
-        for (int nb = 0; nb < G::NB; ++nb) dq[nb] = Half<F16>::mma(frag<F16>(at + nb * 32 * G::TP), dsf, dq[nb]);
+        for (int nb = 0; nb < G::NB; ++nb) dq[nb] = Half<F16>::mma(view.trans(kt, nb, ks), dsf, dq[nb]);
       }
     }
     if (t + 1 < ntiles) store((t + 1) & 1);
     __syncthreads();
   }
   if constexpr (KS > 1) {
-    static_assert(KS == 2 && WAVES * 16 * G::NB * 64 * 4 <= KS * 2 * BUF, "the hand-over reuses the stages");
+    static_assert(KS == 2, "one hand-over");
     float* xo = reinterpret_cast<float*>(smem) + wave * 16 * G::NB * 64 + lane;
     if (ks == 1) {
 #pragma unroll
@@ -615,7 +604,7 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
   typedef typename Half<F16>::x8 X8;
   constexpr bool DV = MODE != 2, DK = MODE != 1;
   constexpr int STATS = 2 * BT * 4;                           // lse * log2(e) and delta of the tile's queries
-  constexpr int BUF = 2 * G::ROWMAJ + 2 * G::TRANS + STATS;   // Q rows, dO rows, Q^T, dO^T, stats
+  constexpr int BUF = 2 * G::TILE + STATS;                    // Q tile, dO tile, stats
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x % GROUP, ks = threadIdx.x / GROUP;
   const int lane = tid & 63, wave = tid >> 6;
@@ -630,6 +619,7 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
   const float* db = p.delta + bh * p.sq;
   const float c2 = p.scale * LOG2E;
   unsigned char* lds = smem + ks * 2 * BUF;
+  const TileView<D, F16> view(lane);
 
   X8 kf[G::C16], vf[DK ? G::C16 : 1];
   {
@@ -648,8 +638,7 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
     if (DV) dv[nb] = zero16();
   }
 
-  TileRegs<D> rq, rg;        // Q rows (scores); dO rows (dP: dK only)
-  TransRegs<D> rqt, rgt;     // Q^T (dK only); dO^T (dV only)
+  TileRegs<D> rq, rg;
   float st = 0.0f;  // one statistic per thread of the group's first wavefront: lse2 (lanes 0-31) or delta (32-63)
   int st_rows = 0;  // rows of the tile it belongs to
   Stream<KS> load(0, p.sq, ks);
@@ -658,9 +647,7 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
     const long long at = (long long)load.first_row() * p.d;
     const int rows = load.rows_left();
     tile_fetch<D>(rq, qb + at, tid, rows, p.d);
-    if (DK) tile_fetch<D>(rg, gb + at, tid, rows, p.d);
-    if (DK) trans_fetch<D>(rqt, qb + at, tid, rows, p.d);
-    if (DV) trans_fetch<D>(rgt, gb + at, tid, rows, p.d);
+    tile_fetch<D>(rg, gb + at, tid, rows, p.d);
     if (tid < 2 * BT) {
       const float* src = tid < BT ? lb : db;  // every lane loads; the factor is applied when stored
       st = src[min(load.first_row() + (tid & (BT - 1)), p.sq - 1)];
@@ -670,14 +657,12 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
   };
   auto store = [&](int buf) {
     unsigned char* base = lds + buf * BUF;
-    tile_store_rows<D>(rq, base, tid);
-    if (DK) tile_store_rows<D>(rg, base + G::ROWMAJ, tid);
-    if (DK) trans_store<D>(rqt, base + 2 * G::ROWMAJ, tid);
-    if (DV) trans_store<D>(rgt, base + 2 * G::ROWMAJ + G::TRANS, tid);
+    tile_store<D>(rq, base, tid, p.d);
+    tile_store<D>(rg, base + G::TILE, tid, p.d);
     if (tid < 2 * BT) {
       float v = tid < BT ? st * LOG2E : st;
       if ((tid & (BT - 1)) >= st_rows) v = tid < BT ? INFINITY : 0.0f;  // a query past the end: probability 0
-      reinterpret_cast<float*>(base + 2 * G::ROWMAJ + 2 * G::TRANS)[tid] = v;
+      reinterpret_cast<float*>(base + 2 * G::TILE)[tid] = v;
     }
   };
   fetch();
@@ -691,17 +676,15 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
   __syncthreads();
   for (int t = 0; t < ntiles; ++t) {
     const unsigned char* qt = lds + (t & 1) * BUF;
-    const unsigned char* gt = qt + G::ROWMAJ;
-    const unsigned char* qtt = qt + 2 * G::ROWMAJ;
-    const unsigned char* gtt = qtt + G::TRANS;
-    const float* stats = reinterpret_cast<const float*>(gtt + G::TRANS);
+    const unsigned char* gt = qt + G::TILE;
+    const float* stats = reinterpret_cast<const float*>(gt + G::TILE);
     if (t + 1 < ntiles) fetch();
     // S and dP: lane = key ln, register i = query 8*(i/4) + 4*kg + i%4 of the tile
     f32x16 s = zero16(), dp = zero16();
 #pragma unroll
     for (int c = 0; c < G::C16; ++c) {
-      s = Half<F16>::mma(frag<F16>(qt + ln * G::RP + (16 * c + 8 * kg) * 2), kf[c], s);
-      if (DK) dp = Half<F16>::mma(frag<F16>(gt + ln * G::RP + (16 * c + 8 * kg) * 2), vf[c], dp);
+      s = Half<F16>::mma(view.rows(qt, c), kf[c], s);
+      if (DK) dp = Half<F16>::mma(view.rows(gt, c), vf[c], dp);
     }
     float pr[16], ds[16];
 #pragma unroll
@@ -718,29 +701,28 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
     }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      const int at = ln * G::TP + (16 * ks + 8 * kg) * 2;
       if constexpr (EXACT) {
         bf16x8 part[3];
         if (DV) {
           parts8<true>(pr + 8 * ks, part);
 #pragma unroll
-          for (int nb = 0; nb < G::NB; ++nb) dv[nb] = mma_exact<F16>(frag<F16>(gtt + at + nb * 32 * G::TP), part, dv[nb]);
+          for (int nb = 0; nb < G::NB; ++nb) dv[nb] = mma_exact<F16>(view.trans(gt, nb, ks), part, dv[nb]);
         }
         if (DK) {
           parts8<false>(ds + 8 * ks, part);
 #pragma unroll
-          for (int nb = 0; nb < G::NB; ++nb) dk[nb] = mma_exact<F16>(frag<F16>(qtt + at + nb * 32 * G::TP), part, dk[nb]);
+          for (int nb = 0; nb < G::NB; ++nb) dk[nb] = mma_exact<F16>(view.trans(qt, nb, ks), part, dk[nb]);
         }
       } else {
         if (DV) {
           const X8 pf = pack8<F16>(pr + 8 * ks);
 #pragma unroll
-          for (int nb = 0; nb < G::NB; ++nb) dv[nb] = Half<F16>::mma(frag<F16>(gtt + at + nb * 32 * G::TP), pf, dv[nb]);
+          for (int nb = 0; nb < G::NB; ++nb) dv[nb] = Half<F16>::mma(view.trans(gt, nb, ks), pf, dv[nb]);
         }
         if (DK) {
           const X8 dsf = pack8<F16>(ds + 8 * ks);
 #pragma unroll
-          for (int nb = 0; nb < G::NB; ++nb) dk[nb] = Half<F16>::mma(frag<F16>(qtt + at + nb * 32 * G::TP), dsf, dk[nb]);
+          for (int nb = 0; nb < G::NB; ++nb) dk[nb] = Half<F16>::mma(view.trans(qt, nb, ks), dsf, dk[nb]);
         }
       }
     }
@@ -748,7 +730,7 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
     __syncthreads();
   }
   if constexpr (KS > 1) {
-    static_assert(KS == 2 && MODE == 0 && WAVES * 32 * G::NB * 64 * 4 <= KS * 2 * BUF, "the hand-over reuses the stages");
+    static_assert(KS == 2 && MODE == 0, "one hand-over of both sums");
     float* xo = reinterpret_cast<float*>(smem) + wave * 32 * G::NB * 64 + lane;
     if (ks == 1) {
 #pragma unroll
@@ -809,27 +791,28 @@ int launch(K kernel, dim3 grid, int threads, int lds, const ChunkTable& tab, con
 template <int D, bool F16, bool EXACT>
 int launch_fwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
   typedef Geo<D> G;
-  constexpr int LDS = 2 * (G::ROWMAJ + G::TRANS);
+  constexpr int LDS = 2 * 2 * G::TILE, SUMS = WAVES * (16 * G::NB + 2) * 64 * 4;  // stages; what a group hands over
+  auto lds = [](int ks) { return std::max(ks * LDS, ks / 2 * SUMS); };
   const dim3 grid((unsigned)jg::cdiv(a.sq, BQ), (unsigned)batch, 1);
   const char* who = "jg_attn_fwd(wide)";
   const int ks = split_of((long long)grid.x * batch, D <= 64 ? 4 : 2);
   if constexpr (D <= 64)
-    if (ks == 4) return launch(&attn_wide_fwd_kernel<D, F16, 4, EXACT>, grid, 4 * GROUP, 4 * LDS, tab, a, s, who);
-  if (ks == 2) return launch(&attn_wide_fwd_kernel<D, F16, 2, EXACT>, grid, 2 * GROUP, 2 * LDS, tab, a, s, who);
+    if (ks == 4) return launch(&attn_wide_fwd_kernel<D, F16, 4, EXACT>, grid, 4 * GROUP, lds(4), tab, a, s, who);
+  if (ks == 2) return launch(&attn_wide_fwd_kernel<D, F16, 2, EXACT>, grid, 2 * GROUP, lds(2), tab, a, s, who);
   return launch(&attn_wide_fwd_kernel<D, F16, 1, EXACT>, grid, GROUP, LDS, tab, a, s, who);
 }
 
 template <int D, bool F16, bool EXACT>
 int launch_bwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
   typedef Geo<D> G;
-  constexpr int DQ_LDS = 2 * (2 * G::ROWMAJ + G::TRANS);
-  constexpr int DKV_LDS = 2 * (2 * G::ROWMAJ + 2 * G::TRANS + 2 * BT * 4);
+  constexpr int DQ_LDS = 2 * 2 * G::TILE, DKV_LDS = 2 * (2 * G::TILE + 2 * BT * 4);  // stages
+  constexpr int SUMS = WAVES * 16 * G::NB * 64 * 4;                                  // what a group hands over of each
   const dim3 dq_grid((unsigned)jg::cdiv(a.sq, BQ), (unsigned)batch, 1);
   const dim3 dkv_grid((unsigned)jg::cdiv(a.sk, BQ), (unsigned)batch, (unsigned)a.nchunks);
   const long long dkv_workgroups = (long long)dkv_grid.x * batch * a.nchunks;
   const char* who = "jg_attn_bwd(wide, dq)";
   int rc = split_of((long long)dq_grid.x * batch, 2) == 2
-               ? launch(&attn_wide_dq_kernel<D, F16, 2, EXACT>, dq_grid, 2 * GROUP, 2 * DQ_LDS, tab, a, s, who)
+               ? launch(&attn_wide_dq_kernel<D, F16, 2, EXACT>, dq_grid, 2 * GROUP, std::max(2 * DQ_LDS, SUMS), tab, a, s, who)
                : launch(&attn_wide_dq_kernel<D, F16, 1, EXACT>, dq_grid, GROUP, DQ_LDS, tab, a, s, who);
   if (rc != JG_OK) return rc;
   who = "jg_attn_bwd(wide, dkv)";
@@ -837,7 +820,7 @@ int launch_bwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_
   // than the chip has CUs, and with EXACT always (register budget, see the kernel)
   if constexpr (D <= (EXACT ? 64 : 96)) {
     if (split_of(dkv_workgroups, 2) == 2)
-      return launch(&attn_wide_dkv_kernel<D, F16, 0, 2, EXACT>, dkv_grid, 2 * GROUP, 2 * DKV_LDS, tab, a, s, who);
+      return launch(&attn_wide_dkv_kernel<D, F16, 0, 2, EXACT>, dkv_grid, 2 * GROUP, std::max(2 * DKV_LDS, 2 * SUMS), tab, a, s, who);
   } else if (EXACT || dkv_workgroups > jg::cu_count()) {
     rc = launch(&attn_wide_dkv_kernel<D, F16, 1, 1, EXACT>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
     if (rc != JG_OK) return rc;
