@@ -546,7 +546,8 @@ int jg_conv_wgrad_framed(void* gw, void* gb, const void* x_frame, const void* x_
  * planes = batch * c_in). Cells of the padded gradient inside the tile go to gx
  * (planes, *size) as `0 + v`; halo cells go to send[slot of the neighbour that
  * owns them] in the layout of jg_halo_pack_3d(from_padded = 1); a NULL slot
- * drops them. Returns JG_ERR_UNSUPPORTED where only the unfused path exists
+ * drops them. Any type and any number of channels, without groups. Returns
+ * JG_ERR_UNSUPPORTED where jg_conv_dgrad runs the direct kernels, which have only the unfused path
  * (workspace as for JG_CONV_DGRAD). Finish with jg_halo_fold_border_3d. */
 int jg_conv_dgrad_fold(void* gx, void* const send[27], const void* w, const void* g,
                        const jg_conv_desc* desc, const jg_halo_geom* geom, int dtype,
