@@ -130,17 +130,18 @@ def _as_64_columns(q, k, chunks: int = 1) -> bool:
     """Whether bf16 heads of fewer than 64 columns against ``chunks`` chunks like ``k`` are better off with zero columns
     up to 64, copies there and back included, on the kernels of that size, which stream their tiles straight into LDS and keep eight
     wavefronts busy a workgroup. Forward / backward, us, own width and as 64 columns: 8 heads x 4096 x 4096 keys, 16 columns
-    119/306 and 69/169, 48 columns 131/333 and 72/178; 32 heads 238/647 and 197/514, 276/754 and 206/560; but 32 heads x 2048 x 2048
-    70/173 and 87/182, 80/204 and 91/196, and 128 heads x 1024 x 2 chunks of 1024 keys 123/329 and 149/374. A width of 32 is a
-    kernel's own, and worth leaving only where its four wavefronts a workgroup leave compute units idle: 8 heads x 4096 x
-    4096 keys 93/237 and 68/173, 16 heads 106/260 and 121/288."""
+    89/170 and 76/172, 32 85/159 and 73/164, 48 105/206 and 81/180; 2 x 8192 x 8192, 32 100/205 and 96/206; 8 x 8192 x 4096, 40 117/317 and 118/288. More rows keep the compute
+    units busy at their own width: 32 heads x 4096, 16 columns 160/358 and 204/494, 48 196/517 and 223/558, 64 heads, 56 432/1078 and
+    457/1131. A width of 32 is a kernel's own, and worth leaving only for the longest sequences."""
     *lead, sq, d = q.shape
     if sq < 2048 or d >= 64 or q.dtype != torch.bfloat16:
         return False
     keys, rows = k.shape[-2] * chunks, math.prod(lead) * sq
     if keys < 4096:
         return False
-    return rows * keys >= 1 << 27 and sq >= 4096 and rows <= 1 << 15 if 24 < d <= 32 else True
+    if 24 < d <= 32:
+        return rows * keys >= 1 << 27 and sq >= 4096 and rows <= 1 << 15
+    return rows <= 1 << 16
 
 
 def _padded_head_size(q, k, bias) -> int:
@@ -260,7 +261,7 @@ def _fused_ok(q, k) -> bool:
     d = q.shape[-1]
     if any(t.data_ptr() % 16 for t in (q, k)):
         return False
-    if _as_64_columns(q, k):  # the merge is a kernel of its own then, 32 heads x 4096 x 4096 keys of 16 columns 187 us, fused 239
+    if _as_64_columns(q, k):  # the merge is a kernel of its own then
         return False
     return d in _F32_MFMA_HEAD_SIZES if q.dtype == torch.float32 else d % 8 == 0 and _mfma16(q, k)
 

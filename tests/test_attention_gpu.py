@@ -647,3 +647,21 @@ def test_narrow_heads_on_long_sequences_run_as_64_columns(h, sq, sk, P, d, dev):
         got = ja.core_backward(dout, q, ks[0], vs[0], out, lse, scale)
         for g, w in zip(got, want):
             assert g.shape == w.shape and rel_l2(g, w) < 2e-2
+
+
+@pytest.mark.parametrize("h,d", [(17, 16), (33, 56)])
+def test_narrow_heads_with_many_rows_keep_their_width(h, d, dev):
+    """Beyond 2^16 rows the kernels of the heads' own width are the faster ones: their results against those of the same heads
+    with zero columns up to 64, which add nothing. Both round probabilities and results to bf16, twice 2^-8 apart at most."""
+    torch.manual_seed(d)
+    mk = lambda: torch.randn(1, h, 4096, d, device=dev).bfloat16()  # noqa: E731
+    q, k, v, dout = mk(), mk(), mk(), mk()
+    assert not ja._as_64_columns(q, k) and ja._as_64_columns(q[:, :16], k[:, :16])
+    wide = [torch.nn.functional.pad(t, (0, 64 - d)) for t in (q, k, v, dout)]
+    out, lse = ja.ring_forward(q, [k], [v], d**-0.5)
+    out64, lse64 = ja.ring_forward(wide[0], [wide[1]], [wide[2]], d**-0.5)
+    assert rel_l2(out, out64[..., :d]) < 2.0**-7 and rel_l2(lse, lse64) < 1e-5
+    got = ja.ring_backward(dout, q, out, lse, [k], [v], d**-0.5)
+    want = ja.ring_backward(wide[3], wide[0], torch.nn.functional.pad(out, (0, 64 - d)), lse, [wide[1]], [wide[2]], d**-0.5)
+    for g, w in zip((got[0], got[1][0], got[2][0]), (want[0], want[1][0], want[2][0])):
+        assert rel_l2(g, w[..., :d]) < 2.0**-7
