@@ -539,7 +539,6 @@ __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void at
         }
   };
 
-  int buf = 0;
   store_stats(0, 0);
   // The K / V fragments came straight from memory: they are waited for here, once. Left
   // to the first MFMA that reads them, the wait would sit inside the loop, behind the
@@ -547,14 +546,19 @@ __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void at
 #pragma unroll
   for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(kf[c]), "+v"(vf[c]));
   __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
+  auto advance = [&](int t, int buf) __attribute__((always_inline)) {
     const bool has_next = t + 1 < ntiles;
     if (has_next) issue_loads(t + 1, buf ^ 1);
     compute_tile(buf);
     if (has_next) store_stats(t + 1, buf ^ 1);
     __syncthreads();
-    buf ^= 1;
+  };
+  int t = 0;
+  for (; t + 1 < ntiles; t += 2) {  // a buffer is then a constant offset of the LDS reads (8 heads x 4096 x 4 chunks 304 -> 297 us)
+    advance(t, 0);
+    advance(t + 1, 1);
   }
+  if (t < ntiles) advance(t, 0);
 
   // combine the two query halves, then write dK / dV (lane = key)
   float* xo = reinterpret_cast<float*>(smem) + kb * (64 * 64);

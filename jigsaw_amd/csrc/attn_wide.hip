@@ -29,8 +29,8 @@
 //                  and Q tiles.
 //
 // A transposed copy of the tile beside it, fetched and written a second time, had these kernels at (copy : transpose reads, with the loads
-// above; forward / dQ / dK and dV, us) 6 heads x 4050 x 4 chunks, head size 80 460 / 559 / 931 : 339 / 357 / 366; 24 x 1000 x 2, 128
-// 65 / 83 / 125 : 60 / 65 / 110; 24 x 739 x 5, 32 54 / 62 / 52 : 48 / 46 / 31; 8 x 4096 x 2, fp16 64 193 / 240 / 195 : 186 / 173 / 161. What is
+// above and two tiles a round; forward / dQ / dK and dV, us) 6 heads x 4050 x 4 chunks, head size 80 460 / 559 / 931 : 312 / 336 / 366; 24 x 1000 x 2, 128
+// 65 / 83 / 125 : 57 / 61 / 106; 24 x 739 x 5, 32 54 / 62 / 52 : 45 / 43 / 30; 8 x 4096 x 2, fp16 64 193 / 240 / 195 : 165 / 156 / 161. What is
 // left is one chain per wavefront, scores, exponentials, products, with two wavefronts a SIMD to fill its gaps.
 //
 // Reference behaviour restated here:
@@ -341,8 +341,8 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
 #pragma unroll
     for (int c = 0; c < G::C16; ++c) asm volatile("" : "+v"(qf[c]));
     __syncthreads();
-    for (int t = 0; t < ntiles; ++t) {
-      const unsigned char* kt = lds + (t & 1) * BUF;
+    auto tile = [&](int t, int buf) __attribute__((always_inline)) {
+      const unsigned char* kt = lds + buf * BUF;
       const unsigned char* vt = kt + G::TILE;
       if (t + 1 < ntiles) fetch();
       // S^T: lane = query ln, register i = key 8*(i/4) + 4*kg + i%4 of the tile
@@ -392,9 +392,15 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
           for (int nb = 0; nb < G::NB; ++nb) o[nb] = Half<F16>::mma(view.trans(vt, nb, ks), pf, o[nb]);
         }
       }
-      if (t + 1 < ntiles) store((t + 1) & 1);
+      if (t + 1 < ntiles) store(buf ^ 1);
       __syncthreads();
+    };
+    int t = 0;
+    for (; t + 1 < ntiles; t += 2) {  // a stage is then a constant offset of the LDS reads (8 heads x 4096 x 2 chunks, 128 287 -> 253 us, fp16 64 184 -> 165)
+      tile(t, 0);
+      tile(t + 1, 1);
     }
+    if (t < ntiles) tile(t, 0);
   }
   // the two lanes of a query saw the same maxima; their sums cover disjoint keys
   l += __shfl_xor(l, 32, 64);
@@ -528,8 +534,8 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
 #pragma unroll
   for (int c = 0; c < G::C16; ++c) asm volatile("" : "+v"(qf[c]), "+v"(dof[c]));
   __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
-    const unsigned char* kt = lds + (t & 1) * BUF;
+  auto tile = [&](int t, int buf) __attribute__((always_inline)) {
+    const unsigned char* kt = lds + buf * BUF;
     const unsigned char* vt = kt + G::TILE;
     if (t + 1 < ntiles) fetch();
     f32x16 s = zero16(), dp = zero16();
@@ -560,9 +566,15 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
         for (int nb = 0; nb < G::NB; ++nb) dq[nb] = Half<F16>::mma(view.trans(kt, nb, ks), dsf, dq[nb]);
       }
     }
-    if (t + 1 < ntiles) store((t + 1) & 1);
+    if (t + 1 < ntiles) store(buf ^ 1);
     __syncthreads();
+  };
+  int t = 0;
+  for (; t + 1 < ntiles; t += 2) {
+    tile(t, 0);
+    tile(t + 1, 1);
   }
+  if (t < ntiles) tile(t, 0);
   if constexpr (KS > 1) {
     static_assert(KS == 2, "one hand-over");
     float* xo = reinterpret_cast<float*>(smem) + wave * 16 * G::NB * 64 + lane;
@@ -674,8 +686,8 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
     if (DK) asm volatile("" : "+v"(vf[c]));
   }
   __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
-    const unsigned char* qt = lds + (t & 1) * BUF;
+  auto tile = [&](int t, int buf) __attribute__((always_inline)) {
+    const unsigned char* qt = lds + buf * BUF;
     const unsigned char* gt = qt + G::TILE;
     const float* stats = reinterpret_cast<const float*>(gt + G::TILE);
     if (t + 1 < ntiles) fetch();
@@ -726,8 +738,18 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
         }
       }
     }
-    if (t + 1 < ntiles) store((t + 1) & 1);
+    if (t + 1 < ntiles) store(buf ^ 1);
     __syncthreads();
+  };
+  int t = 0;
+  if constexpr (D == 96 && MODE == 0) {  // (two tiles a round have no registers left there: 6 heads x 4050 x 4 chunks 366 -> 405 us)
+    for (; t < ntiles; ++t) tile(t, t & 1);
+  } else {
+    for (; t + 1 < ntiles; t += 2) {
+      tile(t, 0);
+      tile(t + 1, 1);
+    }
+    if (t < ntiles) tile(t, 0);
   }
   if constexpr (KS > 1) {
     static_assert(KS == 2 && MODE == 0, "one hand-over of both sums");
