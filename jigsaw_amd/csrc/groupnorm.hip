@@ -3,7 +3,8 @@
 // x is (N, C, S) contiguous (S = product of the local spatial extents); a group is
 // C / G consecutive channels, so the elements of one (sample, group) are one contiguous
 // span. Everything is HBM-bound: 16-byte loads, fp32 accumulation, block partials that a
-// second small kernel adds up in a fixed order (deterministic, no atomics).
+// second small kernel adds up in a fixed order: the same call gives the same bits. (The one atomic, gn_resident_kernel's list,
+// says which launch writes a chunk. Both write it by the same formulas, from the same statistics.)
 //
 // Passes over the tensor. Sharded: forward two (the moments of every group from ONE pass, centred on a
 // sample of the block's own elements; normalise + affine), backward two (the sums; the input
@@ -334,8 +335,40 @@ struct ApplyArgs {
   int C, G;
 };
 
+// y and gx of an element, for every kernel that writes them. The fused products are spelled out: left to the compiler, two
+// kernels may round the same expression differently, and which of two launches writes a chunk depends on timing.
+// x_norm is rounded to the compute dtype and y computed from the rounded value, as the reference computes y from the x_norm tensor.
+// fp16: `rounded` keeps the compiler from one instruction that multiplies, adds and rounds to 16 bits (v_fma_mixlo_f16), which it
+// uses in one kernel and not in the other and which rounds once where fp32 and then fp16 round twice.
+template <int DT>
+__device__ __forceinline__ float rounded(float v) {
+  if (DT == JG_F16) asm("" : "+v"(v));
+  return v;
+}
+template <int DT>
+__device__ __forceinline__ float normalised(float x, float m, float rs) {
+  return Elem<DT>::up(Elem<DT>::down(rounded<DT>((x - m) * rs)));
+}
+template <int DT>
+__device__ __forceinline__ float output(float x_norm, float w, float b) {
+  return rounded<DT>(__builtin_fmaf(x_norm, w, b));
+}
+// rstd (g w - q1 - x_norm q2) with the factors of a row worked out beforehand: three roundings an element (relative error of
+// an fp32 gradient 5.1e-8 where the terms one after the other gave 6.0e-8)
+struct GradFactors {
+  float g, d, one;
+};
+// from_x: elements d = x - mean, otherwise x_norm
+__device__ __forceinline__ GradFactors grad_factors(float rs, float w, float q1, float q2, bool from_x) {
+  return GradFactors{rs * w, from_x ? rs * (rs * q2) : rs * q2, rs * q1};
+}
+template <int DT>
+__device__ __forceinline__ float input_gradient(float g, float d, const GradFactors& f) {
+  return rounded<DT>(__builtin_fmaf(g, f.g, -__builtin_fmaf(d, f.d, f.one)));
+}
+
 // Forward:  x_norm = (x - mean) * rstd, y = x_norm * w[c] + b[c]
-// Backward: gx = rstd * (g * w[c] - gsum / cnt - x_norm * gxsum / cnt); FROM_X: x_norm from x as in the forward
+// Backward: gx = rstd * (g * w[c] - gsum / cnt - x_norm * gxsum / cnt); FROM_X: x_norm from x as in the forward, unrounded
 // for the elements [lo, hi) of a row of channel c, with q1 = gsum / cnt, q2 = gxsum / cnt
 template <int DT, bool BWD, bool FROM_X>
 __device__ __forceinline__ void apply_range(const ApplyArgs& p, int c, float m, float rs, float q1, float q2, long long lo, long long hi, bool vec_ok) {
@@ -348,13 +381,12 @@ __device__ __forceinline__ void apply_range(const ApplyArgs& p, int c, float m, 
   T* out = static_cast<T*>(p.out);
   T* norm = static_cast<T*>(p.out_norm);
   T* kept = static_cast<T*>(p.out_kept);
-  // forward: (y, x_norm): x_norm is rounded to the compute dtype and y computed from the rounded value, as the
-  // reference computes y from the x_norm tensor
-  auto forward = [&](float v, float& xn) {
-    xn = Elem<DT>::up(Elem<DT>::down((v - m) * rs));
-    return xn * w + bv;
+  auto forward = [&](float v, float& xn) {  // (y, x_norm)
+    xn = normalised<DT>(v, m, rs);
+    return output<DT>(xn, w, bv);
   };
-  auto backward = [&](float g, float x) { return rs * (g * w - q1 - (FROM_X ? (x - m) * rs : x) * q2); };
+  const GradFactors f = grad_factors(rs, w, q1, q2, FROM_X);
+  auto backward = [&](float g, float x) { return input_gradient<DT>(g, FROM_X ? x - m : x, f); };
   auto vecs = [&](long long i, long long step, auto count) {
     float v[count()][V], x[count()][V];
 #pragma unroll
@@ -671,10 +703,10 @@ __global__ __launch_bounds__(kThreads, 4) void gn_resident_kernel(ResidentArgs q
   T* kept = static_cast<T*>(p.out_kept);
   const float w = p.weight != nullptr ? Elem<DT>::up(static_cast<const T*>(p.weight)[r.c]) : 1.0f;
   const float bv = !BWD && p.bias != nullptr ? Elem<DT>::up(static_cast<const T*>(p.bias)[r.c]) : 0.0f;
-  const float wr = rs * w, qr = rs * q1, qx = rs * (rs * q2);
+  const GradFactors f = grad_factors(rs, w, q1, q2, true);
   auto result = [&](float v, float x) {
-    if (BWD) return v * wr - ((x - m) * qx + qr);
-    return Elem<DT>::up(Elem<DT>::down((v - m) * rs)) * w + bv;
+    if (BWD) return input_gradient<DT>(v, x - m, f);
+    return output<DT>(normalised<DT>(v, m, rs), w, bv);
   };
   const auto to = buffer_of(out + b0, bytes), to_kept = buffer_of((kept != nullptr ? kept : out) + b0, bytes);
 #pragma unroll

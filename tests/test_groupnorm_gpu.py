@@ -265,6 +265,66 @@ def test_chunks_kept_in_registers(shape, dtype, polls, dev):
     assert (gb - g.double().sum((0, 2))).abs().max() < 1e-5 * scale + 1e-6 * math.sqrt(N * S) * scale
 
 
+def _whole_tensor(shape, dtype, dev):
+    """Inputs of the launches behind ``group_norm`` and a function (polls) -> every tensor that they write."""
+    from jigsaw_amd import _lib
+
+    N, C, G, S = shape
+    gen = torch.Generator(device=dev).manual_seed(4)
+    x, g = (torch.randn(N, C, S, device=dev, generator=gen).add_(0.3).to(dtype) for _ in range(2))
+    w, b = (torch.randn(C, device=dev, generator=gen).to(dtype) for _ in range(2))
+    lib, p, code, nbytes = _lib.load(), _lib.ptr, _lib.dtype_code(dtype), _lib.load().jg_gn_workspace_bytes(N, C, S)
+
+    def run(polls):
+        y, kept, gx = (torch.full_like(x, float("nan")) for _ in range(3))
+        stats, grads = torch.full((2, N, G), float("nan"), device=dev), torch.full((2, C), float("nan"), device=dev)
+        ws, stream = torch.full((nbytes,), 255, dtype=torch.uint8, device=dev), _lib.stream_ptr(dev)
+        assert lib.jg_gn_forward_polls(p(y), p(kept), p(stats[0]), p(stats[1]), p(x), p(w), p(b), N, C, S, G, 1e-5, code, polls, p(ws), nbytes,
+                                       stream) == 0
+        assert lib.jg_gn_backward_polls(p(gx), p(grads[0]), p(grads[1]), p(g), p(x), p(stats[0]), p(stats[1]), p(w), N, C, S, G, code,
+                                        _lib.dtype_code(grads.dtype), polls, p(ws), nbytes, stream) == 0
+        return {"y": y, "kept": kept, "gx": gx, "stats": stats, "grads": grads}
+
+    return run
+
+
+@pytest.mark.parametrize("shape", [
+    (2, 6, 2, 7), (1, 8, 2, 4097), (1, 4, 2, 16385),
+    (1, 8, 1, 9 * 16384 + 5),   # more chunks than every block adds up itself
+    (4, 32, 4, 93300),
+    (1, 64, 2, 16 * 16384),     # the most chunks of a group that wait for each other
+], ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_the_launch_that_writes_a_chunk_does_not_show(shape, dtype, dev):
+    """A chunk whose block gave up waiting (all but a few at one poll) and one whose block did not have the same bits."""
+    run = _whole_tensor(shape, dtype, dev)
+    want = run(256)
+    for polls in (1, 2, 8):
+        for name, t in run(polls).items():
+            assert torch.equal(t, want[name]), f"{name} at {polls} polls"
+
+
+def test_a_busy_chip_does_not_show_in_the_results(dev):
+    """Beside a kernel of another stream that keeps four fifths of the compute units, where blocks do give up, bit for bit what
+    the same call gives alone; and again on the free chip after it."""
+    from jigsaw_amd import attention
+
+    run = _whole_tensor((2, 64, 2, 1 << 18), torch.bfloat16, dev)
+    want = run(128)
+    q, k = (torch.randn(1, 200, n, 64, device=dev).bfloat16() for n in (128, 8192))  # 200 workgroups, about 1 ms a call
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        busy = [attention.ring_forward(q, [k] * 16, [k] * 16, 0.125) for _ in range(3)]
+    got = [run(128) for _ in range(3)]
+    torch.cuda.synchronize()
+    got.append(run(128))
+    assert busy[0][0].isfinite().all()
+    for results in got:
+        for name, t in results.items():
+            assert torch.equal(t, want[name]), name
+
+
 def test_group_norm_in_a_captured_graph(dev):
     """Replays with other inputs, eager work in between, against the eager result."""
     torch.manual_seed(8)
