@@ -434,10 +434,19 @@ __global__ __launch_bounds__(kThreads) void gn_apply_kernel(ApplyArgs p, long lo
 // the two sums), waits for those of the whole (sample, group) and writes its part of y or gx from the registers.
 // The blocks of a unit do run at the same time on a chip that is free, and nothing depends on it: a wait ends after `polls`
 // polls, the block then puts its chunk on a list and is gone, and a second launch, which finds every partial there, reads
-// the chunks of the list again (none, as a rule). Once a block has given up, the others hardly wait.
+// the chunks of the list again (none, as a rule). Once more than half of the blocks have given up, the chip is taken to have
+// less room than a unit needs, where waiting only keeps the rest of the unit away, and the others wait less (kPollsStarved).
 // A partial and the fact that it is there are one 8-byte word, written and read as one (kEmpty: not yet there), so that no
 // fence and no write-back of an L2 lies between the two halves.
 constexpr unsigned long long kEmpty = ~0ull;
+// A poll takes 0.8 us, a wait on a free chip 5 to 30 us: of the 16384 blocks of 8 x 64 x 1024^2 forward none gave up within 96
+// polls, 17 to 180 within 64, a tenth within 48, nine tenths within 8. What more than half of the blocks gave up for has to be
+// longer than that too, or blocks go on giving up by themselves once the chip is free again. Beside a kernel of another stream
+// that holds n compute units for about 3 ms, forward / backward, us (128 and 48 : 256, and 8 for everybody after the first block that
+// gave up); a single chunk on the list took 1.74 / 2.95 ms by the latter rule and takes 0.59 / 0.57:
+//   8 x 64 x 1024^2       n = 0  581 / 569 : 584 / 575   150  971 / 3300 : 972 / 3869   200  2375 / 3737 : 2608 / 3109
+//   2 x 64 x 512^2, 2 groups  0   40 / 50 : 40 / 49      150   92 / 312 : 91 / 348      200   344 / 463 : 286 / 452
+constexpr unsigned kPolls = 128, kPollsStarved = 48;
 constexpr int kMaxPartials = 2 * kThreads;  // partials of a unit: every block of the unit adds them up again
 
 struct ResidentArgs {
@@ -677,7 +686,8 @@ __global__ __launch_bounds__(kThreads, 4) void gn_resident_kernel(ResidentArgs q
 
   __shared__ unsigned long long word_s;
   const bool adds = q.partials <= kDirect || r.k == q.partials - 1;
-  const unsigned polls = __hip_atomic_load(q.left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 && q.polls > 8 ? 8 : q.polls;
+  const unsigned gave_up = __hip_atomic_load(q.left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned polls = gave_up > (blockIdx.x + q.partials) / 2 && q.polls > kPollsStarved ? kPollsStarved : q.polls;
   bool there;
   if (adds) {
     there = held_statistics<DT, BWD>(q, p, r.unit, polls, m, rs, q1, q2);
@@ -1026,9 +1036,6 @@ extern "C" int jg_gn_forward(void* y, float* mean, float* rstd, const void* x, c
   return jg_gn_forward_keep(y, nullptr, mean, rstd, x, weight, bias, batch, channels, spatial, groups, eps, dtype, workspace,
                             workspace_bytes, stream);
 }
-
-// 256 polls of 0.8 us; a wait takes 5 to 30 us on a chip that is free
-static constexpr unsigned kPolls = 256;
 
 extern "C" int jg_gn_forward_keep(void* y, void* x_kept, float* mean, float* rstd, const void* x, const void* weight,
                                   const void* bias, int64_t batch, int64_t channels, int64_t spatial, int64_t groups,

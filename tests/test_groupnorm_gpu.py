@@ -325,6 +325,31 @@ def test_a_busy_chip_does_not_show_in_the_results(dev):
             assert torch.equal(t, want[name]), name
 
 
+def test_blocks_wait_again_once_the_chip_is_free(dev):
+    """What gives up waiting beside a kernel of another stream that leaves less room than a group needs does not send the rest of
+    the tensor, whose blocks have the chip to themselves, through the second launch."""
+    from jigsaw_amd import _lib, attention
+
+    N, C, G, S, chunk = 8, 64, 8, 1 << 20, 32768  # 256 chunks a group; 224 places beside the other kernel
+    lib, p = _lib.load(), _lib.ptr
+    x = torch.randn(N, C, S, device=dev, dtype=torch.bfloat16)
+    y, stats, w = torch.empty_like(x), torch.empty(2, N, G, device=dev), torch.ones(C, device=dev, dtype=torch.bfloat16)
+    nbytes = lib.jg_gn_workspace_bytes(N, C, S)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    q, k = (torch.randn(1, 200, n, 64, device=dev).bfloat16() for n in (128, 8192))
+    side, chunks = torch.cuda.Stream(), N * C * S // chunk
+    for calls in (0, 1, 1):
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            for _ in range(calls):
+                attention.ring_forward(q, [k] * 4, [k] * 4, 0.125)  # about 0.25 ms
+        assert lib.jg_gn_forward(p(y), p(stats[0]), p(stats[1]), p(x), p(w), p(w), N, C, S, G, 1e-5, _lib.dtype_code(x.dtype), p(ws), nbytes,
+                                 _lib.stream_ptr(dev)) == 0
+        torch.cuda.synchronize()
+        left = int(ws.view(torch.int32)[2 * (chunks + N * G)])  # behind a word for every chunk and every group
+        assert left < chunks // 2, f"{left} of {chunks} chunks beside {calls} calls"
+
+
 def test_group_norm_in_a_captured_graph(dev):
     """Replays with other inputs, eager work in between, against the eager result."""
     torch.manual_seed(8)
