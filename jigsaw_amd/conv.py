@@ -404,12 +404,12 @@ def _stuffed(g: torch.Tensor, dense_sp, stride) -> torch.Tensor:
 
 class _Launch:
     """What a direct launch of one layer on one shape needs, worked out once: the descriptor, the workspace and the
-    shape of the result."""
+    shape of the result. ``folds``: the input gradient can be written to its owners, as far as is known."""
 
-    __slots__ = ("desc", "nbytes", "shape", "code")
+    __slots__ = ("desc", "nbytes", "shape", "code", "folds")
 
     def __init__(self, desc, nbytes, shape, code) -> None:
-        self.desc, self.nbytes, self.shape, self.code = desc, nbytes, shape, code
+        self.desc, self.nbytes, self.shape, self.code, self.folds = desc, nbytes, shape, code, True
 
 
 @lru_cache(maxsize=512)
@@ -698,16 +698,22 @@ def conv_nd_input_fold(geom: HaloGeometry, w, g, *, stride=1, padding=0, dilatio
     cell and ``send[offset]`` is the halo block owned by that neighbour (only the
     offsets in ``present``, all by default). ``halo_fold_border_`` finishes the fold
     once the neighbours' blocks have arrived. Returns ``None`` where only the
-    unfused kernels cover the problem. ``out = (gx, send)`` of an earlier call with the same
+    unfused kernels cover the problem, and for every type but bf16, as it always has (the package's own
+    layers go through :func:`_input_fold`, which has no such limit). ``out = (gx, send)`` of an earlier call with the same
     arguments and ``workspace`` are written again instead of new tensors.
     """
+    return _input_fold(geom, w, g, stride, padding, dilation, groups, present, out, workspace, types=(torch.bfloat16,))
+
+
+def _input_fold(geom: HaloGeometry, w, g, stride, padding, dilation, groups, present, out=None, workspace=None, types=tuple(_lib._DTYPES)):
+    """:func:`conv_nd_input_fold` for g of one of ``types``."""
     _lib.require_gpu(w, g)
     n = _check_args(g, w, groups, padding)
     if g.dtype != w.dtype:
         raise RuntimeError(f"grad_output type ({g.dtype}) and weight type ({w.dtype}) should be the same")
     if geom.n_spatial != n:
         raise ValueError(f"geometry has {geom.n_spatial} spatial axes, the convolution {n}")
-    if g.dtype != torch.bfloat16 or groups != 1:  # the fold epilogue exists for ungrouped bf16 layers: say so before sizing a workspace
+    if g.dtype not in types or groups != 1:  # the fold epilogue exists for ungrouped layers: say so before sizing a workspace
         return None
     stride, padding, dilation = _tup(stride, n, "stride"), _tup(padding, n, "padding"), _tup(dilation, n, "dilation")
     g, w = g.contiguous(), w.contiguous()
@@ -720,6 +726,8 @@ def conv_nd_input_fold(geom: HaloGeometry, w, g, *, stride=1, padding=0, dilatio
             f"(expected {(batch, w.shape[0], *out_sp)})"
         )
     launch = _launch_for(1, g.dtype, (batch, c_in, *padded), w.shape, stride, padding, dilation, groups) if workspace is None else None
+    if launch is None and g.dtype != torch.bfloat16 or launch is not None and not launch.folds:
+        return None  # fp16 and fp32 layers that are re-shaped before they reach the kernels; what was declined before
     if launch is not None:
         desc, nbytes, ws = launch.desc, launch.nbytes, _scratch(launch, g.device)
     else:
@@ -741,6 +749,8 @@ def conv_nd_input_fold(geom: HaloGeometry, w, g, *, stride=1, padding=0, dilatio
         _lib.ptr(ws), nbytes, _lib.stream_ptr(g.device),
     )
     if rc == -2:  # only the unfused kernels cover this geometry / dtype
+        if launch is not None:
+            launch.folds = False
         return None
     _lib.check(rc, "jg_conv_dgrad_fold")
     return gx, send
@@ -1140,7 +1150,7 @@ def conv_halo_nway_backward(
     if getattr(config, "fused_fold", False) and config.conv_input_fn is conv_nd_input:
         # dgrad writes the owned cells and the send strips itself; same bits as the
         # three separate steps below
-        fused = conv_nd_input_fold(geom, weight, g, present=present, **kwargs)
+        fused = _input_fold(geom, weight, g, present=present, **kwargs)
         if fused is not None:
             g_x, send = fused
             recv = config.halo_exchange.backward(send) if present else {}

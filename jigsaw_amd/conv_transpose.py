@@ -23,12 +23,12 @@ import torch
 from .conv import (
     _cast_to_autocast_dtype,
     _HipLayerConfig,
+    _input_fold,
     _local_padding,
     _mesh_position,
     _present_offsets,
     conv_nd,
     conv_nd_input,
-    conv_nd_input_fold,
     conv_nd_weight,
 )
 from .halo import HaloGeometry, halo_assemble, halo_fold, halo_fold_border_, halo_pack, neighbour_widths
@@ -125,7 +125,7 @@ def conv_transpose_halo_nway(x, w, b, stride, padding, dilation, spatial_groups,
     geom = transpose_geometry(x.shape[-n:], w.shape[-n:], stride, padding, dilation, ranks, sizes)
     present = _present_offsets(geom, ranks, sizes)
     kwargs = {"stride": stride, "padding": _local_padding(padding, sizes), "dilation": dilation, "groups": int(getattr(config, "groups_local", 1))}
-    fused = conv_nd_input_fold(geom, w, x, present=present, **kwargs) if getattr(config, "fused_fold", False) else None
+    fused = _input_fold(geom, w, x, present=present, **kwargs) if getattr(config, "fused_fold", False) else None
     if fused is not None:
         y, send = fused
         recv = config.halo_exchange.forward(send) if present else {}

@@ -90,6 +90,37 @@ def test_native_and_python_route_of_a_step_agree_bit_for_bit(case, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("case", [c for c in ROUTE_CASES if c[9] == 1 and c[7] > 1], ids=lambda c: f"{c[2]}to{c[3]}_{'x'.join(map(str, c[0]))}_s{c[5]}_mesh{c[7]}")
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_the_python_route_writes_the_input_gradient_to_its_owners_for_every_type(case, dtype, monkeypatch):
+    """Without the native module too: one launch for the input gradient, the tile's part and the strips, with the bits of the
+    separate steps."""
+    size, batch, ci, co, k, s, p, mesh, rank = case[:9]
+    dev, n = torch.device("cuda:0"), len(size)
+    torch.manual_seed(6)
+    kernel, stride, padding, dilation = (k,) * n, (s,) * n, (p,) * n, (1,) * n
+    geom = HaloGeometry.for_conv(size, kernel, stride, padding, dilation, (rank,) * n, (mesh,) * n)
+    mk = lambda *shape: torch.randn(*shape, device=dev).to(dtype)  # noqa: E731
+    present = [o for o in itertools.product((-1, 0, 1), repeat=n) if any(o) and all(0 <= rank + v < mesh for v in o)]
+    strips = [{o: mk(batch, ci, *geom.strip_extent(o, verb)) for o in present} for verb in ("assemble", "fold")]
+    x, w = mk(batch, ci, *size).requires_grad_(), mk(co, ci, *kernel)
+    fold, taken = jc._input_fold, []
+    monkeypatch.setattr(jc, "_step_for", lambda *a: None)
+    monkeypatch.setattr(jc, "_input_fold", lambda *a, **kw: taken.append(fold(*a, **kw)) or taken[-1])
+    res = []
+    for fused in (True, False):
+        held = _Held(*strips)
+        y, _ = jc._ConvNd.apply(x, w, None, stride, padding, dilation, tuple(jc.TileGroup(mesh, rank) for _ in size), None,
+                                jc.HipConvNdConfig.for_rank(n, None, held, fused_fold=fused))
+        torch.manual_seed(7)
+        gx, = torch.autograd.grad(y, x, mk(*y.shape))
+        res.append((gx, *(d[o] for d in held.sent for o in sorted(d))))
+    assert len(taken) == 1 and taken[0] is not None
+    for a, c in zip(*res):
+        assert torch.equal(a, c)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_norms_and_rings_by_the_native_and_the_python_route_agree_bit_for_bit(dtype, monkeypatch):
     from jigsaw_amd import attention, groupnorm, layernorm
