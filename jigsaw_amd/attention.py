@@ -133,6 +133,7 @@ def _as_64_columns(q, k, chunks: int = 1) -> bool:
     89/170 and 76/172, 32 85/159 and 73/164, 48 105/206 and 81/180; 2 x 8192 x 8192, 32 100/205 and 96/206; 8 x 8192 x 4096, 40 117/317 and 118/288. More rows keep the compute
     units busy at their own width: 32 heads x 4096, 16 columns 160/358 and 204/494, 48 196/517 and 223/558, 64 heads, 56 432/1078 and
     457/1131. A width of 32 is a kernel's own, and worth leaving only for the longest sequences."""
+    # (host.cpp's may_want_64_columns asks here about the rows, keys and widths that it names: no others may get a yes)
     *lead, sq, d = q.shape
     if sq < 2048 or d >= 64 or q.dtype != torch.bfloat16:
         return False
@@ -337,6 +338,10 @@ def _resident_forward(q, k_chunks, v_chunks, scale):
         kv = _chunks_as_64_columns(t.to(q.dtype) for t in (*k_chunks, *v_chunks))
         out, lse = _resident_forward(_pad_last(q, 64), kv[:len(k_chunks)], kv[len(k_chunks):], scale)
         return out[..., :q.shape[-1]].contiguous(), lse
+    if q.shape[-1] < 64:  # the module leaves narrow heads on long sequences to the rule above
+        done = _native("ring_forward_at_own_width", q, list(k_chunks), list(v_chunks), scale)
+        if done is not None:
+            return done
     q = _dense(q)
     ks, vs = [_dense(t.to(q.dtype)) for t in k_chunks], [_dense(t.to(q.dtype)) for t in v_chunks]
     batch, sq, d = _flat(q)
@@ -364,6 +369,10 @@ def _resident_backward(dout, q, out, lse, k_chunks, v_chunks, scale):
         dq, dkv = _backward_over(*padded, lse, kv[:P], kv[P:], scale)[:2]
         dk, dv = dkv[..., :d].contiguous().unbind(0)
         return dq[..., :d].contiguous(), list(dk.unbind(0)), list(dv.unbind(0))
+    if q.shape[-1] < 64:  # as in the forward
+        done = _native("ring_backward_at_own_width", dout, q, out, lse, list(k_chunks), list(v_chunks), scale)
+        if done is not None:
+            return done
     dq, _, dks, dvs = _backward_over(dout, q, out, lse, k_chunks, v_chunks, scale)
     return dq, dks, dvs
 

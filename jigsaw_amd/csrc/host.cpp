@@ -263,13 +263,17 @@ constexpr size_t kMostChunks = 16;       // attention._MAX_CHUNKS_PER_CALL
 constexpr int64_t kMostBatch = 65535;    // attention._MOST_BATCH
 constexpr int64_t kMostRows = 1 << 23;   // attention._MOST_ROWS
 
-// What the one-pass kernels take without copies, conversions or zero columns (attention._resident, _as_64_columns)
-bool ring_ok(const at::Tensor& q, const List& k, const List& v, int64_t* batch) {
+// bf16 heads that may be better off with zero columns up to 64: attention._as_64_columns, which has the rule and the figures,
+// decides, and whoever asked it calls the functions `_at_own_width`. Everything for which it can say yes has to be here.
+bool may_want_64_columns(int64_t head_size, int64_t q_rows, int64_t keys) { return head_size < 64 && q_rows >= 2048 && keys >= 4096; }
+
+// What the one-pass kernels take without copies, conversions or zero columns (attention._resident)
+bool ring_ok(const at::Tensor& q, const List& k, const List& v, bool own_width, int64_t* batch) {
   const int64_t n = q.dim();
   if (n < 3 || k.empty() || k.size() > kMostChunks || v.size() != k.size() || q.numel() == 0 || k[0].numel() == 0) return false;
   const int64_t d = q.size(-1), sq = q.size(-2), sk = k[0].dim() == n ? k[0].size(-2) : 0;
   if ((q.scalar_type() != at::kBFloat16 && q.scalar_type() != at::kHalf) || d % 8 != 0 || d > 128 || sq > kMostRows || sk > kMostRows) return false;
-  if (q.scalar_type() == at::kBFloat16 && d < 64 && sq >= 2048 && sk * (int64_t)k.size() >= 4096) return false;
+  if (!own_width && q.scalar_type() == at::kBFloat16 && may_want_64_columns(d, sq, sk * (int64_t)k.size())) return false;
   *batch = q.numel() / (sq * d);
   if (*batch > kMostBatch || !on_gpu(q) || !aligned(q)) return false;
   for (int64_t a = 0; a < n; ++a)
@@ -286,9 +290,10 @@ void addresses(const List& from, P* to) {
   for (size_t j = 0; j < from.size(); ++j) to[j] = from[j].data_ptr();
 }
 
+template <bool OWN_WIDTH>
 py::object ring_forward(const at::Tensor& q, const List& k, const List& v, double scale, uintptr_t stream) {
   int64_t batch;
-  if (!ring_ok(q, k, v, &batch)) return py::none();
+  if (!ring_ok(q, k, v, OWN_WIDTH, &batch)) return py::none();
   at::AutoDispatchBelowADInplaceOrView below;
   const at::Tensor out = at::empty_like(q), lse = at::empty(q.sizes().slice(0, q.dim() - 1), q.options().dtype(at::kFloat));
   const void *kp[kMostChunks], *vp[kMostChunks];
@@ -300,10 +305,11 @@ py::object ring_forward(const at::Tensor& q, const List& k, const List& v, doubl
   return py::make_tuple(out, lse);
 }
 
+template <bool OWN_WIDTH>
 py::object ring_backward(const at::Tensor& dout, const at::Tensor& q, const at::Tensor& out, const at::Tensor& lse, const List& k,
                          const List& v, double scale, uintptr_t stream) {
   int64_t batch;
-  if (!ring_ok(q, k, v, &batch)) return py::none();
+  if (!ring_ok(q, k, v, OWN_WIDTH, &batch)) return py::none();
   for (const at::Tensor* t : {&dout, &out})
     if (t->sizes() != q.sizes() || t->scalar_type() != q.scalar_type() || t->device() != q.device() || !t->is_contiguous() || !aligned(*t)) return py::none();
   if (lse.scalar_type() != at::kFloat || lse.device() != q.device() || !lse.is_contiguous() || lse.sizes() != q.sizes().slice(0, q.dim() - 1))
@@ -447,8 +453,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       .def("forward", &Step::forward)
       .def("backward", &Step::backward)
       .def("finish", &Step::finish);
-  m.def("ring_forward", &ring_forward);
-  m.def("ring_backward", &ring_backward);
+  m.def("may_want_64_columns", &may_want_64_columns);
+  m.def("ring_forward", &ring_forward<false>);
+  m.def("ring_forward_at_own_width", &ring_forward<true>);
+  m.def("ring_backward", &ring_backward<false>);
+  m.def("ring_backward_at_own_width", &ring_backward<true>);
   m.def("ln_partial", &ln_partial);
   m.def("ln_recentre", &ln_recentre);
   m.def("ln_apply", &ln_apply);

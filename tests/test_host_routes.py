@@ -185,3 +185,42 @@ def test_the_native_route_declines_what_needs_a_copy():
     x = torch.randn(4, 6, device=dev)
     assert host.ln_partial(x.t(), False, stream) is None and host.ln_partial(x.double(), False, stream) is None
     assert host.gn_forward(x.half(), 2, torch.ones(6, device=dev), None, 1e-5, False, stream) is None  # another type
+
+
+def test_the_native_route_asks_about_every_head_that_may_be_better_off_as_64_columns():
+    """The rule for zero columns has one place, ``attention._as_64_columns``; the native module takes no such head unasked."""
+    from jigsaw_amd import attention
+
+    may = _lib.host().may_want_64_columns
+    yes = 0
+    for d, sq, sk, P, lead in itertools.product((8, 16, 24, 32, 40, 56, 64, 96), (1024, 2040, 2048, 4096, 8192), (512, 2048, 4096, 4104),
+                                                (1, 2, 4, 16), ((1, 1), (1, 8), (2, 16), (4, 64))):
+        q, k = torch.empty(*lead, sq, d, dtype=torch.bfloat16, device="meta"), torch.empty(*lead, sk, d, dtype=torch.bfloat16, device="meta")
+        wants = attention._as_64_columns(q, k, P)
+        yes += wants
+        assert may(d, sq, sk * P) or not wants, (d, sq, sk, P, lead)
+    assert yes > 50 and not may(32, 128, 256)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(40, 2048, 32), (33, 2048, 48)], ids=str)
+def test_narrow_heads_with_many_rows_take_the_native_route(shape, monkeypatch):
+    from jigsaw_amd import attention
+
+    heads, n, d = shape
+    dev = torch.device("cuda:0")
+    torch.manual_seed(2)
+    q, dout, *kv = (torch.randn(1, heads, n, d, device=dev).bfloat16() for _ in range(6))
+    assert not attention._as_64_columns(q, kv[0], 2)
+
+    def run():
+        out, lse = attention.ring_forward(q, kv[:2], kv[2:], 0.2)
+        dq, dk, dv = attention.ring_backward(dout, q, out, lse, kv[:2], kv[2:], 0.2)
+        return [out, lse, dq, *dk, *dv]
+
+    with monkeypatch.context() as m:
+        m.setattr(attention, "_pointers", None)  # the Python route's pointer tables
+        native = run()
+    monkeypatch.setattr(_lib, "host", lambda: None)
+    for a, c in zip(native, run(), strict=True):
+        assert torch.equal(a, c)
