@@ -379,14 +379,6 @@ int jg_gn_forward(void* y, float* mean, float* rstd, const void* x, const void* 
 int jg_gn_forward_keep(void* y, void* x_kept, float* mean, float* rstd, const void* x, const void* weight, const void* bias,
                        int64_t batch, int64_t channels, int64_t spatial, int64_t groups, float eps, int dtype,
                        void* workspace, size_t workspace_bytes, void* stream);
-/* jg_gn_forward_keep and jg_gn_backward as they are but for `polls`: how often a block asks for the rest of its group before
- * it leaves its part to a second launch (1: nearly always; 0: separate launches, which read the tensors twice). */
-int jg_gn_forward_polls(void* y, void* x_kept, float* mean, float* rstd, const void* x, const void* weight, const void* bias,
-                        int64_t batch, int64_t channels, int64_t spatial, int64_t groups, float eps, int dtype, unsigned polls,
-                        void* workspace, size_t workspace_bytes, void* stream);
-int jg_gn_backward_polls(void* gx, void* gw, void* gb, const void* g, const void* x, const float* mean, const float* rstd,
-                         const void* weight, int64_t batch, int64_t channels, int64_t spatial, int64_t groups, int dtype,
-                         int grad_dtype, unsigned polls, void* workspace, size_t workspace_bytes, void* stream);
 int jg_gn_backward(void* gx, void* gw, void* gb, const void* g, const void* x, const float* mean, const float* rstd,
                    const void* weight, int64_t batch, int64_t channels, int64_t spatial, int64_t groups, int dtype,
                    int grad_dtype, void* workspace, size_t workspace_bytes, void* stream);

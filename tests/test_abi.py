@@ -41,6 +41,13 @@ def test_binding_table_matches_header():
     assert sorted(_lib.SIGNATURES) == declared_symbols()
 
 
+def test_the_interface_holds_no_entry_points_of_the_tests():
+    """What only tests call is bound apart from the header's entry points."""
+    declared = declared_symbols()
+    assert not [s for s in declared if s.endswith("_polls")]
+    assert set(_lib._NOT_IN_THE_HEADER) == {"jg_gn_forward_polls", "jg_gn_backward_polls"} and not set(_lib._NOT_IN_THE_HEADER) & set(declared)
+
+
 def test_abi_version_and_error_string():
     assert jigsaw_amd.abi_version() >= 1
     assert isinstance(jigsaw_amd.load().jg_last_error(), bytes)
