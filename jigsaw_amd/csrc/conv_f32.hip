@@ -422,19 +422,26 @@ int launch(Params p, const Strips& strips, bool fold, hipStream_t s, const char*
 
 namespace jg {
 
-// Every direction of a layer has the same answer.
+// Every direction of a layer has the same answer, so that none is less exact than the others.
 bool f32_conv_supported(const ConvGeom& g, int dtype) {
   if (dtype != JG_F32 || g.groups != 1 || g.batch <= 0 || g.k[0] != 1 || g.in[0] != 1 || g.k[1] != 3 || g.k[2] != 3) return false;
   for (int a = 0; a < 3; ++a)
     if (g.s[a] != 1 || g.d[a] != 1 || g.p[a] > g.k[a] - 1 || g.out[a] < 1) return false;
   const long long tiles = g.batch * ((std::max(g.in[1], g.out[1]) + GR - 1) / GR) * ((std::max(g.in[2], g.out[2]) + TW - 1) / TW);
   if (tiles >= (1ll << 22) || (g.cin + 13) / 14 * ((g.cout + 15) / 16) >= 65536) return false;
-  // Against sums of bf16 parts, forward + both gradients, us (this : that). Up to 16 channels on one side those multiply mostly padding:
+  // Against sums of bf16 parts, forward + both gradients, us (this : that). Up to 16 channels on one side:
   //   4 x 3 -> 16, 256^2 60 : 134   8 x 16 -> 16, 512^2 640 : 708   2 x 12 -> 100, 150^2 154 : 252   8 x 3 -> 64, 512^2 920 : 1829
   // and a layer whose workgroups are fewer than the compute units is bound by its launches:
   //   2 x 24 -> 24, 200^2 108 : 153   1 x 64 -> 64, 100^2 161 : 225   1 x 64 -> 64, 180^2 204 : 250   2 x 48 -> 48, 150^2 193 : 227
   // Beyond, their rate wins:
   //   4 x 20 -> 20, 300^2 249 : 236   2 x 64 -> 64, 180^2 334 : 289   1 x 96 -> 96, 128^2 263 : 243   8 x 64 -> 64, 512^2 6060 : 3851
+  // Within the line the parts are faster in one direction or other of large layers: where 9 to 16 channels go into more than 32
+  // (16 fill the parts' step; this has two stages of 8 and half of its rate), and in the weight gradient of 15 to 21 input channels, which need a
+  // second block of columns here (forward, weight gradient, input gradient):
+  //   8 x 16 -> 128, 256^2 242 : 168, 524 : 509, 342 : 418   8 x 128 -> 16, 256^2 301 : 365, 409 : 491, 305 : 224
+  //   4 x 15 -> 18, 512^2 124 : 111, 287 : 151, 117 : 163    8 x 16 -> 16, 256^2 51 : 66, 91 : 88, 54 : 76
+  // Those directions stay here too: the parts are less exact in all of them. Relative error against float64, 16 -> 128: y 1.6e-7 :
+  // 2.5e-7, gw 6.4e-8 : 2.0e-7, input gradient of 128 from 16 1.6e-7 : 2.5e-7 (3 channels 0.94e-7 : 1.13e-7).
   const int few = std::min(g.cin, g.cout), many = std::max(g.cin, g.cout);
   const long long workgroups = g.batch * ((g.out[1] + TH - 1) / TH) * ((g.out[2] + TW - 1) / TW) * ((many + 31) / 32);
   return few <= 16 || (many <= 64 && workgroups <= cu_count());

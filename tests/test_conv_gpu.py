@@ -868,3 +868,21 @@ def test_fp32_on_the_matrix_instruction(case, dev):
 
     check(*(torch.randint(-3, 4, s, generator=gen).double() for s in shapes), 0, 0, 0)
     check(*(torch.randn(s, generator=gen).double() for s in shapes), 74 + ci // 8, 74 + co // 8, 12)
+
+
+@pytest.mark.parametrize("case", [(2, 16, 128, 70, 131), (2, 128, 16, 66, 100), (1, 15, 18, 150, 200), (3, 12, 48, 90, 70)], ids=str)
+def test_fp32_layers_of_few_channels_are_as_exact_as_their_kernels_in_every_direction(case, dev):
+    """Also the directions that sums of bf16 parts do faster (relative error 2.5e-7 and 1.5e-7 to 3.7e-7 in the weight gradient) keep
+    products and sums in fp32. A chain of n additions whose terms are as large on average is off by 2.5e-8 sqrt(n / 2), 2.5e-8 being
+    what one rounding is off by on average: 1.5e-7 for a stage's 72 products, and a third of that again for what follows; 0.5e-7 for the
+    weight gradient's eight pixels, and as much again for its last roundings."""
+    N, ci, co, h, w_ = case
+    gen = torch.Generator().manual_seed(8)
+    x, w, g = (torch.randn(*s, generator=gen) for s in ((N, ci, h + 2, w_ + 2), (co, ci, 3, 3), (N, co, h, w_)))
+    xd, wd, gd = x.double(), w.double(), g.double()
+    y = jc.conv_nd(x.to(dev), w.to(dev))
+    gx = jc.conv_nd_input(x.shape, w.to(dev), g.to(dev))
+    gw = jc.conv_nd_weight(x.to(dev), w.shape, g.to(dev))
+    assert rel_l2(y, torch.nn.functional.conv2d(xd, wd)) < 2e-7
+    assert rel_l2(gx, torch.nn.grad.conv2d_input(xd.shape, wd, gd)) < 2e-7
+    assert rel_l2(gw, torch.nn.grad.conv2d_weight(xd, wd.shape, gd)) < 1e-7
