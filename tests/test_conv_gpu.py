@@ -604,6 +604,7 @@ def test_fused_dgrad_fold_has_the_bits_of_the_three_steps(case, dev):
 
 
 def test_fused_dgrad_fold_declines_what_the_mfma_kernel_does_not_cover(dev):
+    """The function's own limit: bf16 (the layers reach the kernels of the other types through ``_input_fold``)."""
     from jigsaw_amd.halo import HaloGeometry
 
     geom = HaloGeometry((8, 8), (1, 1), (1, 1))

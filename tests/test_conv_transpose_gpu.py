@@ -163,20 +163,21 @@ def test_grouped_transposed_conv_primitive_equals_torch(dev):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("case", [
-    # tile, C_in, C_out, kernel, stride
-    ((16, 32), 32, 32, (3, 3), (1, 1)), ((13, 21), 5, 3, (3, 3), (1, 1)), ((9, 70), 40, 72, (3, 3), (1, 1)), ((5, 6, 9), 4, 6, (3, 3, 3), (1, 1, 1)),
+    # tile, C_in, C_out, padding, ranks an axis: rank 1 of two has neighbours on one side and raw spans that drift without padding
+    ((16, 32), 32, 32, 1, 3), ((13, 21), 5, 3, 1, 3), ((9, 70), 40, 72, 1, 3), ((5, 6, 9), 4, 6, 1, 3), ((16, 32), 32, 20, 0, 2), ((11, 66), 3, 7, 0, 2),
 ], ids=str)
 def test_raw_output_goes_to_its_owners_for_every_type(case, dtype, dev, monkeypatch):
-    """The rank in the middle of a mesh of three: the raw output written to the tile and the strips by one launch, bit for bit
-    what the separate steps give, for fp16 and fp32 layers as for bf16 ones."""
-    n, cin, cout, k, s = case
+    """The raw output written to the tile and the strips by one launch, bit for bit what the separate steps give, for fp16 and
+    fp32 layers as for bf16 ones."""
+    n, cin, cout, pad, ranks = case
     ns, N = len(n), 2
     torch.manual_seed(5)
-    mesh, rank, p, d = (3,) * ns, (1,) * ns, (1,) * ns, (1,) * ns
+    mesh, rank, k, s, p, d = (ranks,) * ns, (1,) * ns, (3,) * ns, (1,) * ns, (pad,) * ns, (1,) * ns
     x, w = torch.randn(N, cin, *n, device=dev).to(dtype), torch.randn(cin, cout, *k, device=dev).to(dtype)
     geom = jct.transpose_geometry(n, k, s, p, d, rank, mesh)
-    recv = {o: torch.randn(N, cout, *geom.strip_extent(o, "fold"), device=dev).to(dtype) for o in geom.offsets()}
-    groups, taken = tuple(jc.TileGroup(3, 1) for _ in n), []
+    recv = {o: torch.randn(N, cout, *geom.strip_extent(o, "fold"), device=dev).to(dtype) for o in geom.offsets()
+            if neighbour(rank, o, mesh) is not None}
+    groups, taken = tuple(jc.TileGroup(ranks, 1) for _ in n), []
 
     class Exchange:
         def forward(self, send):

@@ -181,7 +181,7 @@ def test_the_native_route_declines_what_needs_a_copy():
         assert host.ring_backward(q, bad_q, q, torch.zeros(2, 3, 64, device=dev), bad_k, bad_k, 1.0, stream) is None
     assert host.ring_backward(q, q, q, torch.zeros(2, 3, 64, device=dev).half(), k, k, 1.0, stream) is None
     assert host.ring_forward(torch.zeros(1, 1, 4096, 32, device=dev).bfloat16(), [torch.zeros(1, 1, 4096, 32, device=dev).bfloat16()] * 2,
-                             [torch.zeros(1, 1, 4096, 32, device=dev).bfloat16()] * 2, 1.0, stream) is None  # better off as 64 columns
+                             [torch.zeros(1, 1, 4096, 32, device=dev).bfloat16()] * 2, 1.0, stream) is None  # attention._as_64_columns is asked first
     x = torch.randn(4, 6, device=dev)
     assert host.ln_partial(x.t(), False, stream) is None and host.ln_partial(x.double(), False, stream) is None
     assert host.gn_forward(x.half(), 2, torch.ones(6, device=dev), None, 1e-5, False, stream) is None  # another type
