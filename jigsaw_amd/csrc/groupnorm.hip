@@ -444,8 +444,9 @@ constexpr unsigned long long kEmpty = ~0ull;
 // longer than that too, or blocks go on giving up by themselves once the chip is free again. Beside a kernel of another stream
 // that holds n compute units for about 3 ms, forward / backward, us (128 and 48 : 256, and 8 for everybody after the first block that
 // gave up); a single chunk on the list took 1.74 / 2.95 ms by the latter rule and takes 0.59 / 0.57:
-//   8 x 64 x 1024^2       n = 0  581 / 569 : 584 / 575   150  971 / 3300 : 972 / 3869   200  2375 / 3737 : 2608 / 3109
-//   2 x 64 x 512^2, 2 groups  0   40 / 50 : 40 / 49      150   92 / 312 : 91 / 348      200   344 / 463 : 286 / 452
+//   8 x 64 x 1024^2           n = 0  580 / 580 : 578 / 581   150  993 / 2409 : 1021 / 3896   200  1675 / 3884 : 2592 / 591 and
+//   (for 20 ms) 1158 / 2508 : 2627 / 3956
+//   2 x 64 x 512^2, 2 groups      0   40 / 49 : 39 / 52      150   89 / 315 : 91 / 342       200   355 / 533 : 293 / 463
 constexpr unsigned kPolls = 128, kPollsStarved = 48;
 constexpr int kMaxPartials = 2 * kThreads;  // partials of a unit: every block of the unit adds them up again
 
