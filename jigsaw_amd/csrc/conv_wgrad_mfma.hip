@@ -18,12 +18,12 @@
 //               channels) shifted by the tap. The kw shift is not 16-byte aligned in
 //               LDS, so a lane reads 10 consecutive pixels once (b128 + b32) and
 //               builds the three kw fragments with funnel shifts.
-//   Workgroup   one wavefront per (g channel block, x channel block, column half);
+//   Workgroup   one wavefront per (g channel block, x channel block, part of the columns or rows of a stage);
 //               it keeps its 9 taps x 32x32 fp32 accumulators in registers for the
 //               whole kernel (144 VGPRs) and walks the pixels. 64->64 2-D: 2x2x2 = 8
 //               wavefronts (two per SIMD, which is what hides the barrier and LDS
 //               write phases); 32->32 3-D: 1x3x2 = 6, plus two that only prefetch.
-//   Stage       2 output rows x 64 columns; consecutive stages of a workgroup walk
+//   Stage       2 output rows x 64 columns (32 at stride 2); consecutive stages of a workgroup walk
 //               down one column strip, so two of the four x rows a stage reads are
 //               the previous stage's last two. The x rows therefore live in a ring of
 //               6 rows per channel in LDS and a stage fetches only its two new rows
@@ -35,7 +35,7 @@
 //               channel-lanes of a fragment read hit distinct banks.
 //   Bias grad   the lanes that carry the g chunks to LDS add them up on the way
 //               (fp32), one partial per workgroup and channel.
-//   Reduction   the two column halves of a pair are added in LDS, the workgroup's partial goes
+//   Reduction   the parts of a pair are added in LDS, the workgroup's partial goes
 //               to the workspace; a second kernel sums the partials in a fixed order
 //               (deterministic) and writes gw in the weight layout and gb, in their own dtype.
 #include <cmath>
@@ -97,12 +97,21 @@ struct WgradParams {
   long long total_stages;  // N * Dout * col_tiles * row_pairs
 };
 
-// Wavefronts per workgroup: (g block, x block) pairs x 2 column halves; a 6-wavefront
-// shape gets two more wavefronts that only help with the prefetch.
-constexpr int HALVES = 2;
+// Wavefronts per workgroup: (g block, x block) pairs x parts of a stage's pixels. Blocks of 64 x 64 and those of a
+// volume have two parts, the halves of the columns; a 6-wavefront shape gets two more wavefronts that only help with the prefetch.
+// Blocks with one or two pairs have four, at stride 1 the quarters of the columns, at stride 2 halves of each row: with two
+// parts there was one wavefront a SIMD, and what it did between its matrix instructions (loads, moves to LDS, the barrier)
+// nothing ran beside; a part's fewer fragments leave room for two (200 to 240 registers, 300 to 320 before).
+// Partials and their reduction included: 2 x 40 -> 72 of 217 x 301 bf16 51 -> 44 us, 4 x 32 -> 64 of 512 x 512 80 -> 73, 7 x 5 -> 118
+// of 229 x 380 92 -> 83, at stride 2 of 6 x 91 -> 23 of 244 x 446 76 -> 64 and of 2 x 77 -> 211 of 436 x 84 80 -> 57; the smallest
+// layers (2 x 20 -> 33 of 100 x 150, 23 us) wait for the setup, the partials and the second launch, as before.
+constexpr int wgrad_parts(int cgb, int cxb) { return cgb * cxb <= 2 ? 4 : 2; }
 constexpr int wgrad_threads(int cgb, int cxb) {
-  return (cgb * cxb * HALVES > 4) ? 512 : 64 * cgb * cxb * HALVES;
+  const int waves = cgb * cxb * wgrad_parts(cgb, cxb);
+  return waves > 4 ? 512 : 64 * waves;
 }
+// Workgroups of one pair fit a compute unit twice.
+constexpr int wgrad_waves_per_simd(int cgb, int cxb) { return wgrad_parts(cgb, cxb) == 4 || wgrad_threads(cgb, cxb) == 512 ? 2 : 1; }
 
 // sum of the 8 values of a chunk
 template <bool F16>
@@ -134,7 +143,7 @@ __device__ __forceinline__ float sum_of_8(const u32x4& v) {
 // stages): the kernel is built without the element-wise border path, and its stage loop loads and
 // stores without conditions.
 template <int CGB, int CXB, int EVEN, bool FRAMED, bool F16 = false, bool ALLIN = false, int ST = 1>
-__global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(WgradParams p) {
+__global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, CXB)) void wgrad3x3_mfma_kernel(WgradParams p) {
   constexpr int THREADS = wgrad_threads(CGB, CXB);
   constexpr int LEAD = EVEN == 2 ? 1 : 0;
   static_assert(!(FRAMED && EVEN != 1), "the framed input is read with even windows only");
@@ -142,20 +151,23 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
   constexpr int SW = Stage<ST>::SW, XR = Stage<ST>::XR, NEW = Stage<ST>::NEW, RING = Stage<ST>::RING;
   constexpr int G_CH = Stage<ST>::G_CH, X_CH = Stage<ST>::X_CH;
   constexpr int G_CPR = SW / 8;  // chunks per g row
-  constexpr int CWAVES = CGB * CXB * HALVES;  // wavefronts that own accumulators
+  constexpr int PARTS = wgrad_parts(CGB, CXB);
+  constexpr int COL_PARTS = ST == 1 ? PARTS : 2, ROW_PARTS = PARTS / COL_PARTS;
+  constexpr int CWAVES = CGB * CXB * PARTS;  // wavefronts that own accumulators
   constexpr int GC = 32 * CGB, XC = 32 * CXB;
   constexpr int G_BYTES = GC * G_CH;          // one g buffer
   constexpr int G_CHUNKS = GC * SR * G_CPR;
   constexpr int XP_CHUNKS = XC * NEW * X_CPR;   // the new x rows of a stage
-  constexpr int CHUNKS = G_CHUNKS + XP_CHUNKS;
+  // Rounds of loads, a chunk a thread: those of g first (the last of them may leave lanes over), then those of x
+  constexpr int G_ROUNDS = (G_CHUNKS + THREADS - 1) / THREADS, X_FIRST = G_ROUNDS * THREADS;
+  constexpr int CHUNKS = X_FIRST + XP_CHUNKS;
   constexpr int ROUNDS = (CHUNKS + THREADS - 1) / THREADS;
-  static_assert(G_CHUNKS % THREADS == 0, "a load round holds g chunks or x chunks, never both");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   unsigned char* const lds_x = smem + 2 * G_BYTES;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kgp = lane >> 5;
-  const int pair = wave % (CGB * CXB), half = (wave / (CGB * CXB)) % HALVES;
+  const int pair = wave % (CGB * CXB), part = (wave / (CGB * CXB)) % PARTS;
   const int cb = pair / CXB, ib = pair % CXB;
 
   // contiguous range of stages for this workgroup; stage -> (n, d, column tile, row pair),
@@ -201,8 +213,8 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
       const int che = ch < cout_valid ? ch : cout_valid - 1;  // a channel past the last one reads the last
       c_goff[rd] = (uint32_t)((che * g_cs + (size_t)r * p.Wout + c8 * 8) * 2);
       c_lds[rd] = (uint32_t)(ch * G_CH + r * (SW * 2) + c8 * 16);
-    } else if (q < CHUNKS) {
-      const int qx = q - G_CHUNKS;
+    } else if (q >= X_FIRST && q < CHUNKS) {
+      const int qx = q - X_FIRST;
       const int c8 = qx % X_CPR;
       const int rr = qx / X_CPR;
       const int r2 = rr % NEW, ch = rr / NEW;   // ch = kd * CIN_B + ci
@@ -238,8 +250,8 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     for (int rd = 0; rd < ROUNDS; ++rd) {
       const int q = tid + rd * THREADS;
       c_toff[rd] = 0;
-      if (q >= G_CHUNKS && q < CHUNKS) {
-        const int qx = q - G_CHUNKS;
+      if (q >= X_FIRST && q < CHUNKS) {
+        const int qx = q - X_FIRST;
         const int c8 = qx % X_CPR, rr = qx / X_CPR;
         const int r2 = rr & 1, ch = rr >> 1;
         const int kd = ch / CIN_B, ci = ch - kd * CIN_B;
@@ -380,7 +392,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
 #pragma unroll
           for (int rd = 0; rd < ROUNDS; ++rd) {
             const int q = tid + rd * THREADS;
-            if (q >= G_CHUNKS && q < CHUNKS) {
+            if (q >= X_FIRST && q < CHUNKS) {
               const int dd = dt + (int)((x_kd >> (2 * rd)) & 3u);
               if (dd >= 0 && dd < p.tn_d) {
                 const u32x4 t = v[rd];
@@ -403,7 +415,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     uintptr_t at[ROUNDS];
     uintptr_t t_at = reinterpret_cast<uintptr_t>(x_org) + t_goff;
 #pragma unroll
-    for (int rd = 0; rd < ROUNDS; ++rd) at[rd] = reinterpret_cast<uintptr_t>((rd + 1) * THREADS <= G_CHUNKS ? g_org : x_org) + c_goff[rd];
+    for (int rd = 0; rd < ROUNDS; ++rd) at[rd] = reinterpret_cast<uintptr_t>(rd < G_ROUNDS ? g_org : x_org) + c_goff[rd];
     if (!inside) {
       // A stage at an edge. A chunk is read wherever its bytes lie inside its tensor, also past the end of its
       // row; store_loads clears the pixels that are not the row's. A chunk without any pixel of the tensor reads
@@ -431,13 +443,13 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
         const uintptr_t safe = reinterpret_cast<uintptr_t>(p.part);
 #pragma unroll
         for (int rd = 0; rd < ROUNDS; ++rd) {
-          const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;
+          const bool g_round = rd < G_ROUNDS;
           const int q = tid + rd * THREADS;
           bool row_ok;
           if (g_round) {
             row_ok = oh0 + (q / G_CPR) % SR < p.Hout;
           } else {
-            const int rr = (q - G_CHUNKS) / X_CPR;
+            const int rr = (q - X_FIRST) / X_CPR;
             const int row = ih0 + rr % NEW, dd = id0 + (rr / NEW) / CIN_B;
             row_ok = q < CHUNKS && row >= 0 && row < p.Hin && dd >= 0 && dd < p.Din;
           }
@@ -458,7 +470,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     }
 #pragma unroll
     for (int rd = 0; rd < ROUNDS; ++rd) {
-      const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;  // THREADS divides G_CHUNKS
+      const bool g_round = rd < G_ROUNDS;
       if (!want_g && g_round) continue;
       v[rd] = jg::load_16_bytes_at(EVEN == 0 ? at[rd] & ~(uintptr_t)3 : at[rd]);
       if (EVEN == 0) {
@@ -481,7 +493,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     };
 #pragma unroll
     for (int rd = 0; rd < ROUNDS; ++rd) {
-      const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;
+      const bool g_round = rd < G_ROUNDS;
       if ((!have_g && g_round) || ((sg.over >> rd) & 1u) == 0) continue;
       const void* begin = g_round ? p.g : p.x;
       const char* end = g_round ? p.g_end : p.x_end;
@@ -523,7 +535,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
 #pragma unroll
     for (int rd = 0; rd < ROUNDS; ++rd) {
       const int q = tid + rd * THREADS;
-      const bool g_round = (rd + 1) * THREADS <= G_CHUNKS;
+      const bool g_round = rd < G_ROUNDS;
       if (g_round && !have_g) continue;
       u32x4 val = sg.v[rd];
       if (EVEN == 0) {
@@ -541,7 +553,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
         val.w &= (g_round ? g_keep[3] : x_keep[3]) & row;
       }
       if (g_round) {
-        *reinterpret_cast<u32x4*>(smem + gbuf * G_BYTES + c_lds[rd]) = val;
+        if (G_CHUNKS % THREADS == 0 || q < G_CHUNKS) *reinterpret_cast<u32x4*>(smem + gbuf * G_BYTES + c_lds[rd]) = val;
         if (bias_part != nullptr) bsum[rd] += counted ? sum_of_8<F16>(val) : 0.0f;
       } else if (q < CHUNKS) {
         int slot = slot0 + (int)((x_row >> (2 * rd)) & 3u);
@@ -580,26 +592,28 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.0f;
 
-  // one 16-pixel column group (cgi = 0 or 1 of this wavefront's half) of a stage whose
-  // four x rows sit in ring rows base .. base + 3 (mod RING): first all its LDS reads
+  // one 16-pixel column group (cgi = 0 or 1 of this wavefront's part) of a stage whose
+  // x rows sit in ring rows base .. base + XR - 1 (mod RING): first all its LDS reads
   // (read_group), then its matrix instructions (mfma_group), so that a stage can ask for both
   // of its groups before the first matrix instruction and meets the LDS latency once.
-  constexpr int GROUPS = SW / 16 / HALVES;
+  constexpr int GROUPS = SW / 16 / COL_PARTS;
+  constexpr int PR = SR / ROW_PARTS, PXR = ST * (PR - 1) + 3;  // output rows of a part, x rows it reads
   struct Frags {
-    u32x4 a[SR];
-    u32x4 d[XR];
-    uint32_t d4[XR], d5[XR];
-    u32x4 odd[XR];  // stride 2
+    u32x4 a[PR];
+    u32x4 d[PXR];
+    uint32_t d4[PXR], d5[PXR];
+    u32x4 odd[PXR];  // stride 2
   };
+  const int row0 = ROW_PARTS == 1 ? 0 : part / COL_PARTS;  // first output row of the part
   auto read_group = [&](Frags& f, int gbuf, int base, int cgi) __attribute__((always_inline)) {
     const unsigned char* gb = smem + gbuf * G_BYTES + (cb * 32 + ln) * G_CH + kgp * 16;
     const unsigned char* xb = lds_x + (ib * 32 + ln) * X_CH + kgp * 16;
-    const int cg = half * GROUPS + cgi;  // 16-pixel column group of this wavefront
+    const int cg = part % COL_PARTS * GROUPS + cgi;  // 16-pixel column group of this wavefront
 #pragma unroll
-    for (int r = 0; r < SR; ++r) f.a[r] = *reinterpret_cast<const u32x4*>(gb + r * (SW * 2) + cg * 32);
+    for (int r = 0; r < PR; ++r) f.a[r] = *reinterpret_cast<const u32x4*>(gb + (row0 + r) * (SW * 2) + cg * 32);
 #pragma unroll
-    for (int rho = 0; rho < XR; ++rho) {
-      int slot = base + rho;
+    for (int rho = 0; rho < PXR; ++rho) {
+      int slot = base + ST * row0 + rho;
       if (slot >= RING) slot -= RING;
       f.d[rho] = *reinterpret_cast<const u32x4*>(xb + slot * X_ROW + cg * 32);
       f.d4[rho] = *reinterpret_cast<const uint32_t*>(xb + slot * X_ROW + cg * 32 + 16);
@@ -609,11 +623,11 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     }
   };
   auto mfma_group = [&](Frags& f) __attribute__((always_inline)) {
-    bf16x8 a[SR];
+    bf16x8 a[PR];
 #pragma unroll
-    for (int r = 0; r < SR; ++r) a[r] = __builtin_bit_cast(bf16x8, f.a[r]);
+    for (int r = 0; r < PR; ++r) a[r] = __builtin_bit_cast(bf16x8, f.a[r]);
 #pragma unroll
-    for (int rho = 0; rho < XR; ++rho) {
+    for (int rho = 0; rho < PXR; ++rho) {
       u32x4 d = f.d[rho];
       uint32_t d4 = f.d4[rho], d5 = f.d5[rho];
       // The values are made opaque so that the kw = 2 fragment below is built with register
@@ -635,7 +649,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
       const bf16x8 b1 = __builtin_bit_cast(bf16x8, ST == 2 ? f.odd[rho] : LEAD ? s2 : s1);
       const bf16x8 b2 = __builtin_bit_cast(bf16x8, ST == 2 ? s1 : LEAD ? s3 : s2);
 #pragma unroll
-      for (int r = 0; r < SR; ++r) {
+      for (int r = 0; r < PR; ++r) {
         const int kh = rho - ST * r;
         if (kh >= 0 && kh < 3) {
           if (F16) {
@@ -663,11 +677,14 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     Staged stg;
     int gbuf = 0, base = 0;
     Cursor c_next = decode(s_begin);  // stage whose loads are issued next
-    issue_loads(stg, c_next, true, 1);
     constexpr int OLD = XR - NEW;  // rows a stage shares with the one above
-    store_loads(stg, true, 0, OLD);
-    issue_loads(stg, c_next, false, 0);
-    store_loads(stg, false, 0, (OLD - NEW + RING) % RING);
+    {
+      Staged top;  // both sets of loads under way at once
+      issue_loads(stg, c_next, true, 1);
+      issue_loads(top, c_next, false, 0);
+      store_loads(stg, true, 0, OLD);
+      store_loads(top, false, 0, (OLD - NEW + RING) % RING);
+    }
     {
       // The loads of a stage are issued, and the registers of the stage before stored, in EVERY
       // stage: the cursor stops at the workgroup's last stage, which the last two stages fetch
@@ -734,7 +751,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
 #pragma unroll
     for (int rd = 0; rd < ROUNDS; ++rd) {
       const int q = tid + rd * THREADS;
-      if (rd * THREADS < G_CHUNKS) {  // rounds that hold g chunks (whole rounds: THREADS divides G_CHUNKS)
+      if (rd < G_ROUNDS) {
         float s = bsum[rd];
 #pragma unroll
         for (int off = SR * G_CPR / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
@@ -743,36 +760,42 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB)) void wgrad3x3_mfma_kernel(
     }
   }
 
-  // Partial of this workgroup. The two column halves of a pair meet in LDS first (the stage buffers are free:
-  // a barrier closed the last stage), three taps at a time, which halves what goes to memory and comes back.
-  // A lane's 16 values of a tap leave as four 16-byte pieces, [tap9][pair][4][lane][4].
-  static_assert(CGB * CXB * 3 * 4096 <= 2 * G_BYTES + XC * X_CH, "three taps of every pair fit the stage buffers");
-  float* const meet = reinterpret_cast<float*>(smem) + pair * 3 * 1024 + lane * 4;
+  // Partial of this workgroup. The parts of a pair meet in LDS first (the stage buffers are free: a barrier closed the last
+  // stage), three taps at a time, the upper half of them with the lower and so on, which leaves one of them to go to memory and
+  // come back. A lane's 16 values of a tap leave as four 16-byte pieces, [tap9][pair][4][lane][4].
+  static_assert(CGB * CXB * (PARTS / 2) * 3 * 4096 <= 2 * G_BYTES + XC * X_CH, "three taps of half of the parts fit the stage buffers");
   float* const out = p.part + slot * (size_t)(9 * GC * XC) + pair * 1024 + lane * 4;
 #pragma unroll
-  for (int kh = 0; kh < 3; ++kh) {
-    if (wave < CWAVES && half == 1) {
+  for (int kh = 0; kh < 3; ++kh)
 #pragma unroll
-      for (int kw = 0; kw < 3; ++kw)
+    for (int step = PARTS / 2; step > 0; step /= 2) {
+      float* const meet = reinterpret_cast<float*>(smem) + (pair * (PARTS / 2) + part % step) * 3 * 1024 + lane * 4;
+      if (wave < CWAVES && part >= step && part < 2 * step) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          *reinterpret_cast<f32x4*>(meet + kw * 1024 + j * 256) =
-              f32x4{acc[kh][kw][4 * j], acc[kh][kw][4 * j + 1], acc[kh][kw][4 * j + 2], acc[kh][kw][4 * j + 3]};
+        for (int kw = 0; kw < 3; ++kw)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            *reinterpret_cast<f32x4*>(meet + kw * 1024 + j * 256) =
+                f32x4{acc[kh][kw][4 * j], acc[kh][kw][4 * j + 1], acc[kh][kw][4 * j + 2], acc[kh][kw][4 * j + 3]};
+      }
+      __syncthreads();
+      if (wave < CWAVES && part < step) {
+#pragma unroll
+        for (int kw = 0; kw < 3; ++kw)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            f32x4 v = *reinterpret_cast<const f32x4*>(meet + kw * 1024 + j * 256);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] += acc[kh][kw][4 * j + k];
+            if (step == 1)
+              *reinterpret_cast<f32x4*>(out + (size_t)(kh * 3 + kw) * (GC * XC) + j * 256) = v;
+            else
+#pragma unroll
+              for (int k = 0; k < 4; ++k) acc[kh][kw][4 * j + k] = v[k];
+          }
+      }
+      __syncthreads();
     }
-    __syncthreads();
-    if (wave < CWAVES && half == 0) {
-#pragma unroll
-      for (int kw = 0; kw < 3; ++kw)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          f32x4 v = *reinterpret_cast<const f32x4*>(meet + kw * 1024 + j * 256);
-#pragma unroll
-          for (int k = 0; k < 4; ++k) v[k] += acc[kh][kw][4 * j + k];
-          *reinterpret_cast<f32x4*>(out + (size_t)(kh * 3 + kw) * (GC * XC) + j * 256) = v;
-        }
-    }
-    __syncthreads();
-  }
 }
 
 // gw = sum over the partials of a block of channels (its workgroups, and in split mode its part pairs, which

@@ -838,6 +838,17 @@ def test_weight_gradient_at_the_ends_of_rows(case, dtype, dev):
     assert torch.equal(gw.cpu(), want.to(dtype)) and torch.equal(gb.cpu(), g.sum((0, 2, 3)).to(dtype))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [
+    # batch, c_in, c_out, padded size, stride: blocks of one and two pairs, whose wavefronts share a stage's columns and rows: rows that
+    # end inside each quarter, one row of a stage's two, more stages than workgroups
+    (1, 32, 32, (3, 18), 1), (1, 64, 32, (4, 35), 1), (2, 32, 64, (5, 51), 1), (1, 64, 24, (130, 258), 1), (3, 8, 50, (67, 195), 1),
+    (1, 32, 32, (3, 33), 2), (1, 64, 32, (5, 32), 2), (2, 32, 64, (9, 37), 2), (1, 50, 24, (131, 261), 2), (3, 96, 32, (66, 130), 2),
+], ids=str)
+def test_weight_gradient_of_narrow_blocks(case, dtype, dev):
+    test_weight_gradient_at_the_ends_of_rows(case, dtype, dev)
+
+
 @pytest.mark.parametrize("case", [
     # batch, c_in, c_out, size of x, padding: 8 x 64 tiles of the outputs (4 x 64 in the weight gradient), stages of 8 channels, blocks of
     # 16 and 32 produced channels, 7 or 14 input channels of the weight gradient, rows that are whole cache lines
