@@ -399,12 +399,19 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
 
   // ---- weights and bias. With one group the weights stay in LDS for the life of the
   // workgroup; with more (many input channels) group g is loaded before the stages that
-  // contract its channels.
+  // contract its channels. They go to LDS without passing through registers, all of a wavefront's transfers under way at once
+  // and, at the start, beside the first stage's loads: 28 to 74 KB a workgroup register by register, and the stage behind them,
+  // were 4 to 6 us before the first product, 2 to 4 now. 4 x 48 -> 48 of 256 x 256 forward 27.4 -> 25.3 us, 2 x 40 -> 72 of
+  // 217 x 301 input gradient 37.3 -> 34.4, 1 x 70 -> 55 of 69 x 38 forward (two groups) 32.4 -> 28.5. (The second stage's loads there too,
+  // in registers of their own: no faster, and spills.) transfers_landed() before the barrier behind which they are read.
   auto load_weights = [&](int grp) {
-    const u32x4* src = p.wprep + ((size_t)blockIdx.y * p.ngroups + grp) * w_slots;
-    for (int i = tid; i < w_slots; i += THREADS) lds_w[i] = src[i];
+    const char* const src = reinterpret_cast<const char*>(p.wprep + ((size_t)blockIdx.y * p.ngroups + grp) * w_slots);
+    typedef __attribute__((address_space(3))) unsigned char* lds_bytes;
+    const uint32_t lds_at = (uint32_t)(uintptr_t)(lds_bytes)smem;
+    for (int i = __builtin_amdgcn_readfirstlane(wave * 64); i < w_slots; i += THREADS)  // (64 divides the slots)
+      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"((uint32_t)(i + lane) * 16u), "s"(src), "s"(lds_at + (uint32_t)i * 16u) : "memory");
   };
-  if (p.ngroups == 1) load_weights(0);
+  auto transfers_landed = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
   if (tid < MT)
     lds_bias[tid] = (p.bias == nullptr || mt * MT + tid >= p.M) ? 0.0f
                     : p.out_kind == 1 ? reinterpret_cast<const float*>(p.bias)[mt * MT + tid]
@@ -1328,7 +1335,9 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   int buf = 0;
   cursor_enter(0);
   issue_stage();
+  if (p.ngroups == 1) load_weights(0);
   store_stage(0, 0);
+  transfers_landed();
   if (stages > 1) issue_stage();
   __syncthreads();
   int q = 0;
@@ -1344,6 +1353,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
       if (p.ngroups > 1 && wstep == 0) {
         // every wavefront is past the barrier that closed the last stage of the group before
         load_weights(wgroup);
+        transfers_landed();
         __syncthreads();
       }
       const int wstep_next = wstep + 1 == p.wc16 ? 0 : wstep + 1;
