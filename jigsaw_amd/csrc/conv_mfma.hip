@@ -48,6 +48,7 @@
 //               and the result is stored as fp32. (A two-part form of it for fp16 operands
 //               remains in the split kernels and is not dispatched.)
 #include <type_traits>
+#include <utility>
 
 #include "conv_common.h"
 
@@ -106,6 +107,9 @@ struct FwdParams {
   // The staged window starts `lead` (0 / 1) pixels before the first one a tile needs, so that its
   // rows stay 4-byte aligned whatever the parity of pad_w - org_w.
   int org_w, lead;
+  // The first extra_h produced rows and extra_w columns (0, or pad_h / pad_w; org_w is then the same) lie above and left of the
+  // tile grid: the workgroups at tile row / column 0 make them beside their tile, see compute_left and compute_top.
+  int extra_h, extra_w;
   int sw;               // tile order inside a plane: row-major inside bands of sw tile columns, band after band
   int total_tiles;      // N * Dout * tiles_h * tiles_w
   int nc16;             // KD * Cp / 16
@@ -349,7 +353,7 @@ enum Mode { PLAIN = 0, STRIDED = 1, STRIDED_DGRAD = 2 };
 // stride 1; FOLD_ANY: any type, any number of channels, also the strided gradient.
 enum Fold { FOLD_NONE = 0, FOLD_WHOLE = 1, FOLD_ANY = 2 };
 
-template <int MT, bool EVEN, int FOLD, bool FRAMED, bool F16 = false, bool PX = false, int MODE = PLAIN>  // MT = produced channels per workgroup: 32 or 64
+template <int MT, bool EVEN, int FOLD, bool FRAMED, bool F16 = false, bool PX = false, int MODE = PLAIN, bool RIM = false>  // MT = produced channels per workgroup: 32 or 64
 __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips, FwdParams p) {
   static_assert(MODE == PLAIN || (FOLD != FOLD_WHOLE && !FRAMED), "strided layers have neither that fold epilogue nor the framed input");
   static_assert(MODE != STRIDED || !FOLD, "the forward pass has nothing to fold");
@@ -359,6 +363,8 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   constexpr int WROWS = MODE != STRIDED ? 4 : MT / 32;                     // produced rows per wavefront
   constexpr int CB = MODE == STRIDED ? 1 : MODE == STRIDED_DGRAD ? 2 : MT / 32;  // blocks of 32 channels (or phases) per wavefront
   constexpr int WTAPS = MODE == STRIDED_DGRAD ? 6 : TAPS;                  // taps of prepared weights
+  static_assert(!RIM || (FOLD && EVEN && !PX && !FRAMED), "built for the input gradient that goes to its owners");
+  constexpr bool LEFT = RIM, TOP = RIM && MT == 32;  // see compute_left, compute_top
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int w_slots = WTAPS * p.wc16 * 2 * MT;  // 16-byte slots of one group of weights
   u32x4* lds_w = reinterpret_cast<u32x4*>(smem);
@@ -448,12 +454,21 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     const int per_plane = p.tiles_h * p.tiles_w;
     int tq = tile / per_plane;
     int j = tile - tq * per_plane;
+    // With columns or rows beside the grid the tiles at its edge have more to do. The tiles of a plane are turned by one from plane to
+    // plane and its columns from row to row: a workgroup, whose steps are whole rows or whole planes, would else stay at one
+    // place of every plane for its life (2 x 32 -> 32 of 128^3 384 -> 339 us), and in one column, where the rows of a power of two
+    // alias in L2 (8 x 64 -> 64 of 1024 x 1024 931 -> 829 us).
+    if (RIM) j = (j + tq) % per_plane;
     const int band = p.tiles_h * p.sw;          // tiles in a full band
     const int b = j / band;                     // band number; the last one may be narrower
     j -= b * band;
     const int width = min(p.sw, p.tiles_w - b * p.sw);
     c.th = j / width;
     c.tw = b * p.sw + (j - c.th * width);
+    if (RIM) {
+      c.tw += c.th % p.tiles_w;
+      if (c.tw >= p.tiles_w) c.tw -= p.tiles_w;
+    }
     c.od = tq % p.Dout;
     c.n = tq / p.Dout;
     return c;
@@ -480,8 +495,8 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     if (ti >= my_tiles) return;
     const TileCoord tc = coord(tile_of(ti));
     cur.od = tc.od;
-    cur.ih0 = ST * (tc.th * TH) - p.pad_h;
-    cur.iw0 = ST * (tc.tw * TW) + p.org_w - p.pad_w - p.lead;  // (org_w is 0 in the strided modes)
+    cur.ih0 = ST * (tc.th * TH) + (TOP ? p.extra_h : 0) - p.pad_h;
+    cur.iw0 = ST * (tc.tw * TW) + p.org_w - p.pad_w - p.lead;  // (org_w is 0 in the strided forward)
     cur.window_in = cur.ih0 >= 0 && cur.ih0 + IN_ROWS <= p.Hin && cur.iw0 >= 0 && cur.iw0 + p.lead + IN_COLS <= p.Win;
     cur.base = reinterpret_cast<const char*>(p.x) +
                2 * ((ptrdiff_t)((size_t)tc.n * p.Cx * chan_stride) + (ptrdiff_t)cur.ih0 * p.Win + cur.iw0);
@@ -788,6 +803,67 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     }
   };
 
+  // The produced columns left of the tile grid (FwdParams::extra_w): their windows lie in the first columns of the staged rows,
+  // and what lies before these is padding, so that column c has the taps kw >= extra_w - c only. A wavefront takes 16 channels of
+  // one column (or one phase of the strided gradient's first position) of the tile's 16 rows, on 16 x 16 x 16 products:
+  // 3 to 6 a stage, 4 accumulators.
+  f32x4 left;
+  constexpr int LBLOCKS = MT / 16;  // blocks of 16 channels
+  const int lcol = __builtin_amdgcn_readfirstlane(wave / LBLOCKS), lch = __builtin_amdgcn_readfirstlane(wave % LBLOCKS) * 16;
+  auto has_left = [&](const TileCoord& tc) { return LEFT && tc.tw == 0 && lcol < (MODE == STRIDED_DGRAD ? 2 * p.extra_w : p.extra_w); };
+  auto compute_left = [&](int buf, int wstep) __attribute__((always_inline)) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+    const int n = lane & 15, quad = (lane >> 4) & 1;  // pixel row / channel, half of the eight channels of a slot
+    const u32x2* in = reinterpret_cast<const u32x2*>(lds_in + buf * STAGE_SLOTS + kg * (IN_ROWS * ROW_SLOTS) + n * ROW_SLOTS) + quad;
+    const u32x2* wt = reinterpret_cast<const u32x2*>(lds_w + ((size_t)wstep * 2 + kg) * MT + lch + n) + quad;
+    auto product = [&](int tap, int row, int col) __attribute__((always_inline)) {
+      const u32x2 a = wt[2 * (size_t)tap * p.wc16 * 2 * MT], b = in[2 * (row * ROW_SLOTS + in_slot(col))];
+      left = F16 ? __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), left, 0, 0, 0)
+                 : __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), left, 0, 0, 0);
+    };
+    if (MODE == STRIDED_DGRAD) {  // position 0 reads column 0 only (taps t = 1 and 2 of compute_phases, by phase)
+      if ((blockIdx.y & 1) == 0) product(1 + lcol, 0, 0);
+      product(4 + lcol, 1, 0);
+      return;
+    }
+#pragma unroll
+    for (int kw = 0; kw < KW; ++kw)
+      if (lcol + kw >= p.extra_w) {
+#pragma unroll
+        for (int kh = 0; kh < KH; ++kh) product(kh * KW + kw, kh, lcol + kw - p.extra_w);
+      }
+  };
+  // The produced rows above it (FwdParams::extra_h), the same way: row r has the taps kh >= extra_h - r. Wavefronts 0 to 3 take a row
+  // (or phase) and a half of the tile's columns each, 4 and 5 the corner, on the products of the tile itself: 3 or 6 a stage
+  // (strided: 2 or 1), 16 accumulators, for which there are registers with 32 produced channels.
+  f32x16 top;
+  const int trow = __builtin_amdgcn_readfirstlane(wave & 1), tpart = __builtin_amdgcn_readfirstlane(wave >> 1);
+  auto has_top = [&](const TileCoord& tc) {
+    return TOP && tc.th == 0 && p.extra_h != 0 && (MODE == STRIDED_DGRAD || trow < p.extra_h) && (tpart < 2 || (tpart == 2 && tc.tw == 0 && p.extra_w != 0));
+  };
+  auto compute_top = [&](int buf, int wstep) __attribute__((always_inline)) {
+    const u32x4* in = lds_in + buf * STAGE_SLOTS + kg * (IN_ROWS * ROW_SLOTS);
+    const u32x4* wt = lds_w + ((size_t)wstep * 2 + kg) * MT + ln;
+    const int col = tpart < 2 ? 32 * tpart + ln + p.lead : ln - p.extra_w;
+    auto product = [&](int tap, int row, int kw) __attribute__((always_inline)) {
+      const u32x4 a = wt[(size_t)tap * p.wc16 * 2 * MT], v = in[row * ROW_SLOTS + in_slot(max(col + kw, 0))];
+      const u32x4 b = col + kw < 0 ? u32x4{0u, 0u, 0u, 0u} : v;
+      top = F16 ? __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), top, 0, 0, 0)
+                : __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), top, 0, 0, 0);
+    };
+    if (MODE == STRIDED_DGRAD) {
+      if (trow == 0) product(3, 0, 0);
+      product(4 + trow, 0, 1);
+      return;
+    }
+#pragma unroll
+    for (int kw = 0; kw < KW; ++kw)
+#pragma unroll
+      for (int kh = 0; kh < KH; ++kh)
+        if (trow + kh >= p.extra_h) product(kh * KW + kw, trow + kh - p.extra_h, kw);
+  };
+
   // Accumulator lane (ln, kg), register i of block cb: produced channel
   // cb*32 + 8*(i/4) + 4*kg + i%4, pixel column wcol0 + ln.
   auto init_acc = [&]() {
@@ -817,6 +893,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
       }
   };
 
+  const int org_h = TOP ? p.extra_h : 0;  // first produced row of the tile grid
   const size_t plane_o = (size_t)p.Hout * p.Wout;
   const size_t ochan = plane_o * p.Dout;  // elements between produced channels
   // RAGGED: the last tile of produced channels when M is not a multiple of MT (its weight
@@ -892,7 +969,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     const int wsw = (ln >> 2) & 3;
 #pragma unroll
     for (int r = 0; r < WROWS; ++r) {
-      const int oh = tc.th * TH + wrow0 + r;
+      const int oh = tc.th * TH + org_h + wrow0 + r;
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
@@ -947,7 +1024,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
                          (size_t)tw0);
 #pragma unroll
       for (int r = 0; r < WROWS; ++r) {
-        const int oh = tc.th * TH + wrow0 + r;
+        const int oh = tc.th * TH + org_h + wrow0 + r;
         auto pair = [&](int cb, int i) {
           f32x2 v2 = {acc[cb][r][i], acc[cb][r][i + 1]};
           return F16 ? __builtin_bit_cast(uint32_t, __builtin_convertvector(v2, f16x2))
@@ -966,7 +1043,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
                       4 * (((size_t)tc.n * p.M + (size_t)mt * MT + ch0) * ochan + (size_t)tc.od * plane_o);
 #pragma unroll
       for (int r = 0; r < WROWS; ++r) {
-        const int oh = tc.th * TH + wrow0 + r;
+        const int oh = tc.th * TH + org_h + wrow0 + r;
         if (oh < p.Hout && ow >= 0 && ow < p.Wout) {
           const uint32_t voff = (uint32_t)(4 * ((size_t)(4 * kg) * ochan + (size_t)oh * p.Wout + ow));
           // the channel's base walks by additions (a product per store costs a scalar multiply, a 64-bit add
@@ -987,7 +1064,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     }
 #pragma unroll
     for (int r = 0; r < WROWS; ++r) {
-      const int oh = tc.th * TH + wrow0 + r;
+      const int oh = tc.th * TH + org_h + wrow0 + r;
       if (oh < p.Hout && ow >= 0 && ow < p.Wout) {
         const uint32_t voff = (uint32_t)(2 * ((size_t)(4 * kg) * ochan + (size_t)oh * p.Wout + ow));
         const char* yc = ybase;  // walks by additions, as above
@@ -1012,7 +1089,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   // row has (4-byte stores at 2-byte aligned addresses run at the rate of aligned ones).
   auto epilogue_phases = [&](const TileCoord& tc) {
     const int pa = blockIdx.y & 1;
-    const int iw = 2 * (tc.tw * TW + wcol0 + ln) - p.px_w;
+    const int iw = 2 * (tc.tw * TW + p.org_w + wcol0 + ln) - p.px_w;
     const bool ok0 = iw >= 0 && iw < p.Wx, ok1 = iw + 1 >= 0 && iw + 1 < p.Wx;
     const size_t plane_x = (size_t)p.Hx * p.Wx;
     const int m_left = p.M - mt * MT - 4 * kg;
@@ -1022,7 +1099,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     const uint32_t st = es * (uint32_t)plane_x;
 #pragma unroll
     for (int r = 0; r < WROWS; ++r) {
-      const int ih = 2 * (tc.th * TH + wrow0 + r) + pa - p.px_h;
+      const int ih = 2 * (tc.th * TH + org_h + wrow0 + r) + pa - p.px_h;
       if (ih < 0 || ih >= p.Hx) continue;
       const uint32_t row = 4 * kg * st + es * (uint32_t)(ih * p.Wx + iw);
       auto walk = [&](auto store) __attribute__((always_inline)) {
@@ -1095,7 +1172,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     const int cd = od - (rd == 0 ? 0 : (rd == 1 ? p.lo_d : p.lo_d + p.nD));
     const int ed = rd == 0 ? p.lo_d : (rd == 1 ? p.nD : hi_d);
     const size_t plane0 = (size_t)tc.n * p.M + (size_t)mt * MT;
-    const int th0 = tc.th * TH, tw0 = tc.tw * TW + p.org_w;
+    const int th0 = tc.th * TH + org_h, tw0 = tc.tw * TW + p.org_w;
     // A tile that lies wholly inside the own extent (wave-uniform test): plain rows of
     // the unpadded tile, no per-cell routing.
     if (rd == 1 && th0 >= p.lo_h && th0 + TH <= p.lo_h + p.nH && tw0 >= p.lo_w && tw0 + TW <= p.lo_w + p.nW) {
@@ -1196,7 +1273,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     constexpr bool PHASES = MODE == STRIDED_DGRAD;
     const int pa = PHASES ? blockIdx.y & 1 : 0;
     const int Hp = PHASES ? p.Hx : p.Hout, Wp = PHASES ? p.Wx : p.Wout;  // the produced tensor
-    const int ow = PHASES ? 2 * (tc.tw * TW + wcol0 + ln) - p.px_w : tc.tw * TW + p.org_w + wcol0 + ln;
+    const int ow = PHASES ? 2 * (tc.tw * TW + p.org_w + wcol0 + ln) - p.px_w : tc.tw * TW + p.org_w + wcol0 + ln;
     const int od = tc.od;
     const int rd = od < p.lo_d ? 0 : (od < p.lo_d + p.nD ? 1 : 2);
     const int cd = od - (rd == 0 ? 0 : (rd == 1 ? p.lo_d : p.lo_d + p.nD));
@@ -1239,7 +1316,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     const int blocks = PHASES ? 1 : CB;
 #pragma unroll
     for (int r = 0; r < WROWS; ++r) {
-      const int oh = __builtin_amdgcn_readfirstlane(PHASES ? 2 * (tc.th * TH + wrow0 + r) + pa - p.px_h : tc.th * TH + wrow0 + r);
+      const int oh = __builtin_amdgcn_readfirstlane(PHASES ? 2 * (tc.th * TH + org_h + wrow0 + r) + pa - p.px_h : tc.th * TH + org_h + wrow0 + r);
       if (oh < 0 || oh >= Hp) continue;
       const int rh = region(oh, p.lo_h, p.nH);
       const int ch = oh - (rh == 0 ? 0 : (rh == 1 ? p.lo_h : p.lo_h + p.nH));
@@ -1312,6 +1389,71 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     }
   };
 
+  // The columns left of the tile grid and the rows above it: pixel (oh, ow) and, count of them, channels m0 + step(i) of a lane. One of
+  // oh and ow differs from lane to lane: ALONG_H says which.
+  auto place = [&](const TileCoord& tc, int oh, int ow, auto along_h, int m0, int count, auto channel, auto value) __attribute__((always_inline)) {
+    constexpr bool ALONG_H = decltype(along_h)::value;
+    // (the parameters from the kernel-argument segment: see epilogue_fold_any)
+    typedef const __attribute__((address_space(4))) FwdParams* Args;
+    Args args = nullptr;
+#if defined(__HIP_DEVICE_COMPILE__)
+    args = reinterpret_cast<Args>(reinterpret_cast<uintptr_t>((void*)__builtin_amdgcn_kernarg_segment_ptr()) + sizeof(StripTable));
+    asm volatile("" : "+s"(args));
+#endif
+    const __attribute__((address_space(4))) FwdParams& p = *args;
+    const int Hp = MODE == STRIDED_DGRAD ? p.Hx : p.Hout, Wp = MODE == STRIDED_DGRAD ? p.Wx : p.Wout;  // the produced tensor
+    if (oh < 0 || oh >= Hp || ow < 0 || ow >= Wp) return;
+    const uint32_t es = p.out_kind == 1 ? 4u : 2u;
+    char* base;
+    size_t ps, at;  // elements between channels of the destination, and to the pixel inside a channel
+    if (FOLD) {
+      auto region = [](int v, int lo, int n) { return v < lo ? 0 : (v < lo + n ? 1 : 2); };
+      auto within = [](int v, int r, int lo, int n) { return v - (r == 0 ? 0 : (r == 1 ? lo : lo + n)); };
+      auto extent = [](int r, int lo, int n, int all) { return r == 0 ? lo : (r == 1 ? n : all - lo - n); };
+      const int rd = region(tc.od, p.lo_d, p.nD), rh = region(oh, p.lo_h, p.nH), rw = region(ow, p.lo_w, p.nW);
+      // (wave-uniform indices into the table: see epilogue_fold)
+      constexpr int STEP = ALONG_H ? 3 : 1;
+      const int slot = __builtin_amdgcn_readfirstlane(rd * 9 + (ALONG_H ? rw : 3 * rh)), r = ALONG_H ? rh : rw;
+      char* const low = static_cast<char*>(strip_entry(slot));
+      char* const mid = slot + STEP == 13 ? reinterpret_cast<char*>(p.y) : static_cast<char*>(strip_entry(slot + STEP));
+      char* const high = static_cast<char*>(strip_entry(slot + 2 * STEP));
+      base = r == 0 ? low : (r == 1 ? mid : high);
+      const int eh = extent(rh, p.lo_h, p.nH, Hp), ew = extent(rw, p.lo_w, p.nW, Wp);
+      ps = (size_t)extent(rd, p.lo_d, p.nD, p.Dout) * eh * ew;
+      at = ((size_t)within(tc.od, rd, p.lo_d, p.nD) * eh + within(oh, rh, p.lo_h, p.nH)) * ew + within(ow, rw, p.lo_w, p.nW);
+    } else {
+      base = reinterpret_cast<char*>(p.y);
+      ps = (size_t)p.Dout * Hp * Wp;
+      at = ((size_t)tc.od * Hp + oh) * Wp + ow;
+    }
+    if (base == nullptr) return;
+    const uintptr_t to = reinterpret_cast<uintptr_t>(base) + es * (((size_t)tc.n * p.M + m0) * ps + at);
+#pragma unroll
+    for (int i = 0; i < count; ++i) {
+      if (m0 + channel(i) >= p.M) continue;
+      const uintptr_t d = to + es * ps * channel(i);
+      const float v = value(i);
+      if (p.out_kind == 1) {
+        *reinterpret_cast<JG_GLOBAL float*>(d) = FOLD ? 0.0f + v : v;  // (a sum with zero clears a zero's sign)
+      } else {
+        uint16_t bits = F16 ? __builtin_bit_cast(uint16_t, (_Float16)v) : __builtin_bit_cast(uint16_t, (__bf16)v);
+        if (FOLD && (bits & 0x7fffu) == 0) bits = 0;
+        *reinterpret_cast<JG_GLOBAL uint16_t*>(d) = bits;
+      }
+    }
+  };
+  auto epilogue_left = [&](const TileCoord& tc) {  // a lane holds four neighbouring channels of the pixel in row lane % 16
+    const int row = tc.th * TH + org_h + (lane & 15);
+    place(tc, MODE == STRIDED_DGRAD ? 2 * row + (blockIdx.y & 1) - p.px_h : row, MODE == STRIDED_DGRAD ? lcol - p.px_w : lcol, std::true_type{},
+          mt * MT + lch + 4 * (lane >> 4), 4, [](int i) { return i; }, [&](int i) { return left[i]; });
+  };
+  auto epilogue_top = [&](const TileCoord& tc) {
+    const int pos = tpart < 2 ? tc.tw * TW + p.org_w + 32 * tpart + ln : ln;
+    if (tpart == 2 && ln >= p.extra_w) return;
+    place(tc, MODE == STRIDED_DGRAD ? (int)(blockIdx.y & 1) - p.px_h : trow, MODE == STRIDED_DGRAD ? 2 * pos + trow - p.px_w : pos, std::false_type{},
+          mt * MT + 4 * kg, 16, [](int i) { return 8 * (i >> 2) + (i & 3); }, [&](int i) { return top[i]; });
+  };
+
   // ---- main loop over the stages (tile, 16-channel step) of this workgroup. The
   // global loads of a stage are issued a whole stage ahead: right after the previous
   // stage's registers were written to LDS, in the middle of the stage before.
@@ -1346,8 +1488,14 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     // a wavefront whose 4 x 32 pixels all lie outside the produced tensor (ragged last tiles) only
     // takes part in the staging and the barriers
     const TileCoord tcur = coord(tile_of(ti));
+    const bool left_too = has_left(tcur), top_too = has_top(tcur);
+    if (left_too) left = *reinterpret_cast<const f32x4*>(lds_bias + lch + 4 * (lane >> 4));
+    if (top_too) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) top[i] = lds_bias[8 * (i >> 2) + 4 * kg + (i & 3)];
+    }
     const int wave_col = tcur.tw * TW + p.org_w + wcol0;
-    const bool live = wave_col < p.Wout && wave_col + 32 > 0 && tcur.th * TH + wrow0 < p.Hout;
+    const bool live = wave_col < p.Wout && wave_col + 32 > 0 && tcur.th * TH + org_h + wrow0 < p.Hout;
     int wstep = 0, wgroup = 0;
     for (int c16 = 0; c16 < p.nc16; ++c16, ++q) {
       if (p.ngroups > 1 && wstep == 0) {
@@ -1389,6 +1537,8 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
           compute_kw(buf, wstep, 2, wstep_next);
         }
       }
+      if (left_too) compute_left(buf, wstep);
+      if (top_too) compute_top(buf, wstep);
       __syncthreads();
       buf ^= 1;
       if (++wstep == p.wc16) {
@@ -1403,6 +1553,8 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     if constexpr (FOLD == FOLD_ANY) epilogue_fold_any(tcur, buf ^ 1);
     else if constexpr (FOLD == FOLD_WHOLE) epilogue_fold(tcur, buf ^ 1);
     else epilogue(tcur, buf ^ 1);
+    if (left_too) epilogue_left(tcur);
+    if (top_too) epilogue_top(tcur);
   }
 }
 
@@ -1488,8 +1640,9 @@ size_t conv_ws_bytes(int split, int KD, int C, int M, size_t x_elements, bool ph
 // more rounds of tiles: a chip full of workgroups for each was as many starts (weights, bias, the first stage's
 // latency) on every compute unit, one after the other. 64 -> 128 channels of 4 x 256 x 256 at stride 2 forward 32.7 -> 27.2 us;
 // 96 -> 96 of 4 x 128 x 256 input gradient 62 -> 54 us, 64 -> 128 of 8 x 512 x 512 forward 320 -> 305 us.
+long long cus_per_xcd() { return jg::cu_count() / 8 > 0 ? jg::cu_count() / 8 : 1; }
 int workgroups_for(long long tiles, int mtiles) {
-  const long long cus = jg::cu_count() / 8 > 0 ? jg::cu_count() / 8 : 1;  // of an XCD
+  const long long cus = cus_per_xcd();
   const long long share = (tiles + 7) / 8;                        // tiles of an XCD
   const long long all = share < cus ? share : cus;
   if (mtiles > 1 && mtiles <= cus) {
@@ -1577,12 +1730,11 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
     p.Wout = (L.Wout - 1 + L.px_w) / 2 + 1;
   }
   const int TH = L.mode == STRIDED ? TILE_H / 2 : TILE_H, TW = L.mode == STRIDED ? TILE_W / 2 : TILE_W;
-  p.tiles_h = (p.Hout + TH - 1) / TH;
   // Where to put the tile grid. A tile's staged rows start at input column org_w + TW * tw - pad_w.
   // When the rows of x are a multiple of 128 bytes apart, an origin that makes this a multiple of
   // TW puts every staged row segment on a cache-line boundary (144 bytes: two lines instead of
   // three); it is taken when it costs no extra tile column.
-  p.org_w = 0;
+  p.org_w = p.extra_h = p.extra_w = 0;
   // (not where it would take the 16-byte store path away: a plain 16-bit result with rows of whole pieces)
   const bool wide_rows = !L.fold && L.split != 1 && L.Wout % 8 == 0 && !phases;
   if (!wide_rows && L.mode == PLAIN && L.pad_w % TW != 0 && L.Win % 64 == 0 && (reinterpret_cast<uintptr_t>(x16) & 127) == 0) {
@@ -1591,7 +1743,31 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
   }
   // rows of the staged windows start at even columns where `lead` can see to it: 4-byte aligned loads
   const bool even = (L.Win % 2 == 0) && ((reinterpret_cast<uintptr_t>(x16) & 3) == 0);
+  // The first pad_w columns beside the first tile column and the first pad_h rows beside the first tile row, where that saves a
+  // workgroup a tile: a power of two and its halo are 64 t + 1 or 2 columns wide and 16 u + 1 or 2 rows high, and the last
+  // of their t + 1 tile columns and u + 1 rows cost as much as a whole one (staged rows, barriers) for what little they hold. EXTRA_FIGURES
+  // Rows of x then start at the first staged column, on cache lines where they are whole lines themselves.
+  if (L.fold && even) {
+    auto spare = [](int extent, int pad, int tile) {
+      return (pad == 1 || pad == 2) && extent > pad && (extent - pad + tile - 1) / tile < (extent + tile - 1) / tile ? pad : 0;
+    };
+    auto walk = [&](int eh, int ew) {  // tiles of a workgroup
+      const long long n = (long long)L.N * L.Dout * ((p.Hout - eh + TH - 1) / TH) * ((p.Wout - (ew ? ew : p.org_w) + TW - 1) / TW), share = (n + 7) / 8;
+      const int per = workgroups_for(n, lay.mtiles) / 8;
+      return (share + per - 1) / per * (((long long)per * lay.mtiles + cus_per_xcd() - 1) / cus_per_xcd());
+    };
+    const int eh = MT == 32 ? spare(p.Hout, L.pad_h, TH) : 0, ew = spare(p.Wout, L.pad_w, TW);
+    long long least = walk(0, 0);
+    for (const auto& e : {std::make_pair(0, ew), std::make_pair(eh, 0), std::make_pair(eh, ew)})
+      if (walk(e.first, e.second) < least) {
+        least = walk(e.first, e.second);
+        p.extra_h = e.first;
+        p.extra_w = e.second;
+      }
+    if (p.extra_w) p.org_w = p.extra_w;
+  }
   p.lead = even ? (L.pad_w - p.org_w) & 1 : 0;
+  p.tiles_h = (p.Hout - p.extra_h + TH - 1) / TH;
   p.tiles_w = (p.Wout - p.org_w + TW - 1) / TW;
   p.sw = p.tiles_w;
   const long long tiles = (long long)L.N * L.Dout * p.tiles_h * p.tiles_w;
@@ -1615,12 +1791,22 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
   void (*kern)(StripTable, FwdParams) = nullptr;
   if (L.f16 && L.xt != nullptr)
     JG_FAIL(JG_ERR_UNSUPPORTED, "%s: the framed input is built for bf16 only", who);
+  const bool rim = p.extra_h != 0 || p.extra_w != 0;
   if (L.fold && (L.split || L.f16 || phases || lay.mtiles * MT != L.M)) {
     auto any = [&](auto f16) {
       constexpr bool F = decltype(f16)::value;
-      if (phases) kern = even ? &conv3x3_mfma_kernel<32, true, FOLD_ANY, false, F, false, STRIDED_DGRAD> : &conv3x3_mfma_kernel<32, false, FOLD_ANY, false, F, false, STRIDED_DGRAD>;
-      else if (MT == 64) kern = even ? &conv3x3_mfma_kernel<64, true, FOLD_ANY, false, F> : &conv3x3_mfma_kernel<64, false, FOLD_ANY, false, F>;
-      else kern = even ? &conv3x3_mfma_kernel<32, true, FOLD_ANY, false, F> : &conv3x3_mfma_kernel<32, false, FOLD_ANY, false, F>;
+      if (phases)
+        kern = rim    ? &conv3x3_mfma_kernel<32, true, FOLD_ANY, false, F, false, STRIDED_DGRAD, true>
+               : even ? &conv3x3_mfma_kernel<32, true, FOLD_ANY, false, F, false, STRIDED_DGRAD>
+                      : &conv3x3_mfma_kernel<32, false, FOLD_ANY, false, F, false, STRIDED_DGRAD>;
+      else if (MT == 64)
+        kern = rim    ? &conv3x3_mfma_kernel<64, true, FOLD_ANY, false, F, false, PLAIN, true>
+               : even ? &conv3x3_mfma_kernel<64, true, FOLD_ANY, false, F>
+                      : &conv3x3_mfma_kernel<64, false, FOLD_ANY, false, F>;
+      else
+        kern = rim    ? &conv3x3_mfma_kernel<32, true, FOLD_ANY, false, F, false, PLAIN, true>
+               : even ? &conv3x3_mfma_kernel<32, true, FOLD_ANY, false, F>
+                      : &conv3x3_mfma_kernel<32, false, FOLD_ANY, false, F>;
     };
     if (L.f16) any(std::true_type{});
     else any(std::false_type{});
@@ -1642,8 +1828,14 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
       else strided(std::false_type{}, std::false_type{});
     }
   } else if (L.fold) {
-    if (MT == 64) kern = even ? &conv3x3_mfma_kernel<64, true, FOLD_WHOLE, false> : &conv3x3_mfma_kernel<64, false, FOLD_WHOLE, false>;
-    else kern = even ? &conv3x3_mfma_kernel<32, true, FOLD_WHOLE, false> : &conv3x3_mfma_kernel<32, false, FOLD_WHOLE, false>;
+    if (MT == 64)
+      kern = rim    ? &conv3x3_mfma_kernel<64, true, FOLD_WHOLE, false, false, false, PLAIN, true>
+             : even ? &conv3x3_mfma_kernel<64, true, FOLD_WHOLE, false>
+                    : &conv3x3_mfma_kernel<64, false, FOLD_WHOLE, false>;
+    else
+      kern = rim    ? &conv3x3_mfma_kernel<32, true, FOLD_WHOLE, false, false, false, PLAIN, true>
+             : even ? &conv3x3_mfma_kernel<32, true, FOLD_WHOLE, false>
+                    : &conv3x3_mfma_kernel<32, false, FOLD_WHOLE, false>;
   } else if (L.xt != nullptr) {
     if (MT == 64) kern = even ? &conv3x3_mfma_kernel<64, true, false, true> : &conv3x3_mfma_kernel<64, false, false, true>;
     else kern = even ? &conv3x3_mfma_kernel<32, true, false, true> : &conv3x3_mfma_kernel<32, false, false, true>;

@@ -820,6 +820,24 @@ def test_fused_dgrad_fold_any_channels_types_and_strides(case, dtype, dev):
         assert torch.equal(send[o].view(bits), (want_send[o] + 0).view(bits)), f"strip {o}"
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("case", [
+    # as above, with images enough for several tiles a workgroup: produced tensors one or two rows and columns larger than a whole number
+    # of tiles, which are made beside the tiles at the edge, rows with 32 produced channels only
+    ((16, 64), (1, 1), (1, 1), (0, 0), 1, 200, 32, 16, "all"),
+    ((16, 64), (1, 1), (1, 1), (0, 0), 1, 140, 64, 40, "some"),
+    ((16, 128), (1, 2), (1, 0), (0, 0), 1, 90, 50, 8, "all"),
+    ((32, 64), (0, 1), (1, 1), (1, 0), 1, 150, 20, 16, "all"),
+    ((13, 64), (1, 1), (1, 1), (0, 0), 1, 280, 7, 24, "all"),     # columns only, the tile row not full
+    ((16, 30), (1, 1), (1, 1), (0, 0), 1, 300, 32, 16, "all"),    # rows only
+    ((3, 16, 64), (1, 1, 1), (1, 1, 1), (0, 0, 0), 1, 40, 32, 8, "all"),
+    ((32, 128), (1, 1), (0, 0), (0, 0), 2, 60, 40, 16, "all"),
+    ((32, 256), (0, 1), (1, 0), (1, 0), 2, 40, 33, 24, "some"),
+], ids=str)
+def test_rows_and_columns_beside_the_tile_grid(case, dtype, dev):
+    test_fused_dgrad_fold_any_channels_types_and_strides(case, dtype, dev)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("case", [
     # batch, c_in, c_out, padded size, stride: row ends inside a stage's window, with the tensors' ends behind them and not
