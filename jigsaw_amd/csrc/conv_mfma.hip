@@ -47,6 +47,7 @@
 //               channel groups; the contraction runs over the six part products that matter
 //               and the result is stored as fp32. (A two-part form of it for fp16 operands
 //               remains in the split kernels and is not dispatched.)
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -1569,21 +1570,25 @@ struct Layout {
 
 int pad16(int c) { return (c + CK - 1) / CK * CK; }
 
+// Whether tiles of 64 produced channels pad no further than those of 32 do; the strided input gradient has tiles of 32 only.
+bool may_take_64(int M, bool phases) { return (M + 31) / 32 * 32 % 64 == 0 && !phases; }
+
 // K: contraction length with the channels padded to a multiple of 16 per depth tap. phases: the strided
 // input gradient, tiles of 32 channels twice (one for each phase row), six taps each.
-Layout layout_of(int K, int M, bool phases = false) {
+Layout layout_of(int K, int M, bool phases, int MT) {
   Layout L;
   const int taps = phases ? 6 : TAPS;
   const int mpad = (M + 31) / 32 * 32;
-  L.MT = (mpad % 64 == 0 && !phases) ? 64 : 32;
+  L.MT = MT;
   L.mtiles = mpad / L.MT * (phases ? 2 : 1);
   L.nc16 = K / CK;
   const size_t budget = 160 * 1024 - 2 * (size_t)STAGE_BYTES - L.MT * 4;
   int cap = (int)(budget / ((size_t)taps * 2 * L.MT * 16));
   if (cap < 1) cap = 1;
-  L.wc16 = L.nc16 < cap ? L.nc16 : cap;
+  L.ngroups = (L.nc16 + cap - 1) / cap;
+  if (L.ngroups < 1) L.ngroups = 1;
+  L.wc16 = (L.nc16 + L.ngroups - 1) / L.ngroups;
   if (L.wc16 < 1) L.wc16 = 1;
-  L.ngroups = (L.nc16 + L.wc16 - 1) / L.wc16;
   const size_t slots = (size_t)taps * L.wc16 * 2 * L.MT;
   L.prep_bytes = (size_t)L.mtiles * L.ngroups * slots * 16;
   L.lds_bytes = slots * 16 + 2 * (size_t)STAGE_BYTES + L.MT * 4;
@@ -1631,7 +1636,9 @@ size_t split_bytes(size_t elements, int parts) { return (elements * parts * 2 + 
 size_t conv_ws_bytes(int split, int KD, int C, int M, size_t x_elements, bool phases) {
   const SplitSpec sp = split_spec(split);
   const bool joined = joined_blocks(split, KD, C);
-  const size_t prep = layout_of(joined ? KD * pad16(sp.nblk * C) : sp.nblk * KD * pad16(C), M, phases).prep_bytes;
+  const int K = joined ? KD * pad16(sp.nblk * C) : sp.nblk * KD * pad16(C);
+  size_t prep = layout_of(K, M, phases, 32).prep_bytes;
+  if (may_take_64(M, phases)) prep = std::max(prep, layout_of(K, M, phases, 64).prep_bytes);
   return split ? (prep + 255) / 256 * 256 + split_bytes(x_elements, joined ? sp.nblk : sp.parts) : prep;
 }
 
@@ -1666,6 +1673,66 @@ int split_launch(uint16_t* dst, const SRC* src, size_t batch, size_t per_batch, 
   return JG_OK;
 }
 
+// The tile grid of a launch: produced channels a tile, origin and what lies beside it (FwdParams::org_w, extra_h, extra_w).
+struct Tiling {
+  int MT, org_w, extra_h, extra_w;
+};
+
+// Hout, Wout: produced cells, or positions of the strided input gradient. wide_rows: 16-bit rows of whole 16-byte pieces.
+Tiling tiling_of(const Launch& L, int Hout, int Wout, bool wide_rows, bool even, bool on_lines) {
+  const int TH = L.mode == STRIDED ? TILE_H / 2 : TILE_H, TW = L.mode == STRIDED ? TILE_W / 2 : TILE_W;
+  const bool phases = L.mode == STRIDED_DGRAD;
+  // Where to put the tile grid. A tile's staged rows start at input column org_w + TW * tw - pad_w.
+  // When the rows of x are a multiple of 128 bytes apart, an origin that makes this a multiple of
+  // TW puts every staged row segment on a cache-line boundary (144 bytes: two lines instead of
+  // three); it is taken when it costs no extra tile column.
+  int org_w = 0;
+  // (not where it would take the 16-byte store path away: a plain 16-bit result with rows of whole pieces)
+  if (!wide_rows && L.mode == PLAIN && L.pad_w % TW != 0 && L.Win % 64 == 0 && on_lines) {
+    const int org = L.pad_w % TW - TW;
+    if ((L.Wout - org + TW - 1) / TW <= (L.Wout + TW - 1) / TW) org_w = org;
+  }
+  // The first pad_w columns beside the first tile column and the first pad_h rows beside the first tile row, where that saves a
+  // workgroup a tile: a power of two and its halo are 64 t + 1 or 2 columns wide and 16 u + 1 or 2 rows high, and the last
+  // of their t + 1 tile columns and u + 1 rows cost as much as a whole one (staged rows, barriers) for what little they hold.
+  // Rows of x then start at the first staged column, on cache lines where they are whole lines themselves. Gradient with the fold
+  // of 2 x 32 -> 32 channels of 128^3 429 -> 338 us (16 tiles a plane for 27), at stride 2 of 4 x 64 -> 128 of 256 x 256 53.5 -> 34.8 (one
+  // tile a workgroup for two), 4 x 32 -> 32 of 256 x 256 26.3 -> 21.6, 8 x 8 -> 24 of 64 x 512 24.9 -> 20.2.
+  auto spare = [](int extent, int pad, int tile) {
+    return (pad == 1 || pad == 2) && extent > pad && (extent - pad + tile - 1) / tile < (extent + tile - 1) / tile ? pad : 0;
+  };
+  auto walk = [&](int MT, int eh, int ew) {  // tiles a compute unit goes through
+    const long long n = (long long)L.N * L.Dout * ((Hout - eh + TH - 1) / TH) * ((Wout - (ew ? ew : org_w) + TW - 1) / TW), share = (n + 7) / 8;
+    const int mtiles = (L.M + MT - 1) / MT * (phases ? 2 : 1);
+    const long long per = std::max(1, workgroups_for(n, mtiles) / 8);
+    return (share + per - 1) / per * ((per * mtiles + cus_per_xcd() - 1) / cus_per_xcd());
+  };
+  // 64 produced channels a tile where they pad no further than 32 and the tiles go round: a tile of 32 takes 0.55 to 0.65 of the time of
+  // one of 64 (the same rows staged, half of the products; 0.8 in the strided forward, whose tiles hold fewer), and where the chip is not
+  // full twice as many of them run beside each other. Forward of 2 x 64 -> 64 of 128 x 128 24.2 -> 17.0 us, 1 x 64 -> 64 of 256 x 256
+  // 24.9 -> 18.2, 2 x 128 -> 128 of 128 x 128 39 -> 27, 1 x 70 -> 55 of 69 x 38 32 -> 21; gradient with the fold of 4 x 64 -> 64 of 256 x 256
+  // (512 tiles of 32 with the rows and columns beside them for 340 of 64) 50 -> 42. Forced, where the chip is full: 4 x 64 -> 64 of
+  // 256 x 256 forward 30.5 -> 33.2, 5 x 49 -> 59 of 586 x 314 105 -> 120. Tiles at the edge take about a tenth longer for rows above them.
+  Tiling best{};
+  double least = 0.0;
+  for (const int MT : {64, 32}) {
+    if (MT == 64 && !may_take_64(L.M, phases)) continue;
+    if (MT == 32 && L.xt != nullptr && least > 0.0) continue;
+    const int eh = L.fold && even && MT == 32 ? spare(Hout, L.pad_h, TH) : 0, ew = L.fold && even ? spare(Wout, L.pad_w, TW) : 0;
+    const double tile = MT == 64 ? 1.0 : L.mode == STRIDED ? 0.8 : 0.65;
+    bool taken = least == 0.0;
+    for (const auto& e : {std::make_pair(0, 0), std::make_pair(0, ew), std::make_pair(eh, 0), std::make_pair(eh, ew)}) {
+      const double cost = (double)walk(MT, e.first, e.second) * tile * (e.first ? 1.1 : 1.0);
+      if (least == 0.0 || cost < (taken ? least : 0.9 * least)) {
+        least = cost;
+        best = Tiling{MT, e.second ? e.second : org_w, e.first, e.second};
+        taken = true;
+      }
+    }
+  }
+  return best;
+}
+
 int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const char* who) {
   const SplitSpec sp = split_spec(L.split);
   const bool joined = joined_blocks(L.split, L.KD, L.C);
@@ -1681,8 +1748,15 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
     JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, ws_bytes, need);
   JG_REQUIRE((reinterpret_cast<uintptr_t>(ws) & 15) == 0, "%s: workspace must be 16-byte aligned",
              who);
-  const Layout lay = layout_of(K, L.M, phases);
-  const int MT = lay.MT;
+  // the produced cells, or the positions (i, j) of the strided input gradient
+  const int Hout = phases ? (L.Hout - 1 + L.px_h) / 2 + 1 : L.Hout, Wout = phases ? (L.Wout - 1 + L.px_w) / 2 + 1 : L.Wout;
+  const bool wide_rows = !L.fold && L.split != 1 && L.Wout % 8 == 0 && !phases;
+  const uintptr_t x_at = reinterpret_cast<uintptr_t>(L.split ? ws : L.x);  // (the parts of a split x lie a multiple of 256 bytes behind ws)
+  // rows of the staged windows start at even columns where `lead` can see to it: 4-byte aligned loads
+  const bool even = L.Win % 2 == 0 && (x_at & 3) == 0;
+  const Tiling til = tiling_of(L, Hout, Wout, wide_rows, even, (x_at & 127) == 0);
+  const int MT = til.MT;
+  const Layout lay = layout_of(K, L.M, phases, MT);
   uint16_t* wprep = static_cast<uint16_t*>(ws);
   const size_t total_w = lay.prep_bytes / 2;
   JG_REQUIRE(total_w < (1ull << 31), "%s: weight tensor too large", who);
@@ -1723,49 +1797,16 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
   p.Dout = L.Dout; p.Hout = L.Hout; p.Wout = L.Wout;
   p.pad_d = L.pad_d; p.pad_h = L.pad_h; p.pad_w = L.pad_w;
   p.Hx = p.Wx = p.px_h = p.px_w = 0;
-  if (phases) {  // the kernel's grid runs over the positions (i, j)
+  if (phases) {  // the kernel's grid runs over the positions
     p.Hx = L.Hout; p.Wx = L.Wout;
     p.px_h = L.px_h; p.px_w = L.px_w;
-    p.Hout = (L.Hout - 1 + L.px_h) / 2 + 1;
-    p.Wout = (L.Wout - 1 + L.px_w) / 2 + 1;
+    p.Hout = Hout;
+    p.Wout = Wout;
   }
   const int TH = L.mode == STRIDED ? TILE_H / 2 : TILE_H, TW = L.mode == STRIDED ? TILE_W / 2 : TILE_W;
-  // Where to put the tile grid. A tile's staged rows start at input column org_w + TW * tw - pad_w.
-  // When the rows of x are a multiple of 128 bytes apart, an origin that makes this a multiple of
-  // TW puts every staged row segment on a cache-line boundary (144 bytes: two lines instead of
-  // three); it is taken when it costs no extra tile column.
-  p.org_w = p.extra_h = p.extra_w = 0;
-  // (not where it would take the 16-byte store path away: a plain 16-bit result with rows of whole pieces)
-  const bool wide_rows = !L.fold && L.split != 1 && L.Wout % 8 == 0 && !phases;
-  if (!wide_rows && L.mode == PLAIN && L.pad_w % TW != 0 && L.Win % 64 == 0 && (reinterpret_cast<uintptr_t>(x16) & 127) == 0) {
-    const int org = L.pad_w % TW - TW;
-    if ((L.Wout - org + TW - 1) / TW <= (L.Wout + TW - 1) / TW) p.org_w = org;
-  }
-  // rows of the staged windows start at even columns where `lead` can see to it: 4-byte aligned loads
-  const bool even = (L.Win % 2 == 0) && ((reinterpret_cast<uintptr_t>(x16) & 3) == 0);
-  // The first pad_w columns beside the first tile column and the first pad_h rows beside the first tile row, where that saves a
-  // workgroup a tile: a power of two and its halo are 64 t + 1 or 2 columns wide and 16 u + 1 or 2 rows high, and the last
-  // of their t + 1 tile columns and u + 1 rows cost as much as a whole one (staged rows, barriers) for what little they hold. EXTRA_FIGURES
-  // Rows of x then start at the first staged column, on cache lines where they are whole lines themselves.
-  if (L.fold && even) {
-    auto spare = [](int extent, int pad, int tile) {
-      return (pad == 1 || pad == 2) && extent > pad && (extent - pad + tile - 1) / tile < (extent + tile - 1) / tile ? pad : 0;
-    };
-    auto walk = [&](int eh, int ew) {  // tiles of a workgroup
-      const long long n = (long long)L.N * L.Dout * ((p.Hout - eh + TH - 1) / TH) * ((p.Wout - (ew ? ew : p.org_w) + TW - 1) / TW), share = (n + 7) / 8;
-      const int per = workgroups_for(n, lay.mtiles) / 8;
-      return (share + per - 1) / per * (((long long)per * lay.mtiles + cus_per_xcd() - 1) / cus_per_xcd());
-    };
-    const int eh = MT == 32 ? spare(p.Hout, L.pad_h, TH) : 0, ew = spare(p.Wout, L.pad_w, TW);
-    long long least = walk(0, 0);
-    for (const auto& e : {std::make_pair(0, ew), std::make_pair(eh, 0), std::make_pair(eh, ew)})
-      if (walk(e.first, e.second) < least) {
-        least = walk(e.first, e.second);
-        p.extra_h = e.first;
-        p.extra_w = e.second;
-      }
-    if (p.extra_w) p.org_w = p.extra_w;
-  }
+  p.org_w = til.org_w;
+  p.extra_h = til.extra_h;
+  p.extra_w = til.extra_w;
   p.lead = even ? (L.pad_w - p.org_w) & 1 : 0;
   p.tiles_h = (p.Hout - p.extra_h + TH - 1) / TH;
   p.tiles_w = (p.Wout - p.org_w + TW - 1) / TW;
@@ -2018,7 +2059,7 @@ int mfma_dgrad(void* gx, const void* w, const void* go, const ConvGeom& g, void*
 int mfma_dgrad_fold(void* gx, void* const strips[27], const int lo[3], const int n[3], const void* w,
                     const void* go, const ConvGeom& g, void* ws, size_t ws_bytes, hipStream_t s, int dtype) {
   // the epilogues address the MT channel planes of a tile through a 32-bit byte offset
-  const int MT = layout_of(g.k[0] * pad16(g.cout), g.cin, g.s[2] == 2).MT, es = dtype == JG_F32 ? 4 : 2;
+  const int MT = may_take_64(g.cin, g.s[2] == 2) ? 64 : 32, es = dtype == JG_F32 ? 4 : 2;
   if ((long long)n[0] * n[1] * n[2] * es * MT >= (1ll << 32) || (long long)g.in[0] * g.in[1] * g.in[2] * es * MT >= (1ll << 32))
     JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_dgrad_fold(mfma): %d planes of the tile do not fit a 32-bit offset", MT);
   return dgrad_launch(gx, strips, lo, n, w, go, g, ws, ws_bytes, s, "jg_conv_dgrad_fold(mfma)", dtype);

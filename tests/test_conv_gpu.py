@@ -829,6 +829,8 @@ def test_fused_dgrad_fold_any_channels_types_and_strides(case, dtype, dev):
     ((16, 128), (1, 2), (1, 0), (0, 0), 1, 90, 50, 8, "all"),
     ((32, 64), (0, 1), (1, 1), (1, 0), 1, 150, 20, 16, "all"),
     ((13, 64), (1, 1), (1, 1), (0, 0), 1, 280, 7, 24, "all"),     # columns only, the tile row not full
+    ((14, 64), (1, 1), (1, 1), (0, 0), 1, 600, 64, 8, "some"),    # the same with 64 produced channels, all and 50 of them there
+    ((14, 64), (1, 1), (1, 1), (0, 0), 1, 600, 50, 8, "all"),
     ((16, 30), (1, 1), (1, 1), (0, 0), 1, 300, 32, 16, "all"),    # rows only
     ((3, 16, 64), (1, 1, 1), (1, 1, 1), (0, 0, 0), 1, 40, 32, 8, "all"),
     ((32, 128), (1, 1), (0, 0), (0, 0), 2, 60, 40, 16, "all"),
@@ -836,6 +838,25 @@ def test_fused_dgrad_fold_any_channels_types_and_strides(case, dtype, dev):
 ], ids=str)
 def test_rows_and_columns_beside_the_tile_grid(case, dtype, dev):
     test_fused_dgrad_fold_any_channels_types_and_strides(case, dtype, dev)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("case", [
+    # batch, c_in, c_out, size, stride: tiles of 64 produced channels (launches that fill the chip) and, with fewer images, of 32; whole
+    # 16-byte rows and others, channels that end inside a tile, more contraction steps than LDS holds weights for
+    (600, 16, 64, (16, 64), 1), (40, 16, 64, (16, 64), 1), (600, 7, 50, (9, 33), 1), (40, 7, 50, (9, 33), 1), (300, 80, 64, (5, 40), 1), (3, 80, 128, (5, 40), 1),
+    (600, 16, 64, (16, 64), 2), (40, 16, 64, (16, 64), 2), (600, 9, 60, (11, 35), 2), (30, 70, 60, (11, 35), 2),
+], ids=str)
+def test_tiles_of_64_and_of_32_channels_exactly(case, dtype, dev):
+    """Whole numbers, as in test_strided_3x3_layers_exactly."""
+    N, ci, co, size, stride = case
+    gen = torch.Generator().manual_seed(9)
+    x = torch.randint(-2, 3, (N, ci, *size), generator=gen).float()
+    w = torch.randint(-1, 2, (co, ci, 3, 3), generator=gen).float()
+    b = torch.randint(-3, 4, (co,), generator=gen).float()
+    want = torch.nn.functional.conv2d(x, w, b, stride=stride, padding=1)  # sums below 2^24: exact in fp32
+    y = jc.conv_nd(x.to(dtype).to(dev), w.to(dtype).to(dev), b.to(dtype).to(dev), stride=stride, padding=1)
+    assert torch.equal(y.cpu(), want.to(dtype))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
