@@ -88,6 +88,8 @@ struct FwdParams {
   const uint16_t* x;    // (N, C, Din, Hin, Win) bf16: the tensor that is convolved
   const char* x_end;    // one past the last byte of x
   const u32x4* wprep;   // prepared weights, [m_tile][group][tap9][wc16][kg][MT][8]
+  const uint16_t* wraw;  // the weights as they are, which each workgroup puts in order itself (arrange_weights); NULL: wprep
+  int transposed;        // (with wraw) as in prep_weights_kernel
   const uint16_t* bias; // (M,) or NULL
   uint16_t* y;          // (N, M, Dout, Hout, Wout)
   int N, C, M;          // batch, channels of x, produced channels
@@ -417,6 +419,68 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     const uint32_t lds_at = (uint32_t)(uintptr_t)(lds_bytes)smem;
     for (int i = __builtin_amdgcn_readfirstlane(wave * 64); i < w_slots; i += THREADS)  // (64 divides the slots)
       asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"((uint32_t)(i + lane) * 16u), "s"(src), "s"(lds_at + (uint32_t)i * 16u) : "memory");
+  };
+  // The same from the weights as they are. raw_weights() puts the workgroup's share into the stage buffers (one run of memory
+  // forward, a run for each contraction channel in the input gradient) and arrange_weights() deals it out from there, a slot of eight
+  // channels and nine taps at a time (72 reads of two bytes and nine stores of sixteen a thread for 64 x 64 channels, 1.5 to 2 us). The
+  // preparation is a launch of 4.7 us less, twice a step, and the host's time for it: 64 -> 128 at stride 2 of 4 x 256 x 256, the step
+  // 144.6 -> 141 us; 2 x 31 -> 39 of 52 x 40 at stride 2 forward 11.7 -> 10.7, 4 x 32 -> 32 of 256 x 256 input gradient 22.3 -> 20.9; with
+  // 64 x 64 channels and one tile a workgroup the kernel's share of it is about what the launch took.
+  const int left_m = min(MT, p.M - mt * MT);     // produced channels of the tile that exist
+  const int taps_m = p.KD * TAPS;                // weights of a pair of channels
+  const int run = p.transposed ? left_m * taps_m : left_m * p.C * taps_m, runs = p.transposed && left_m != p.M ? p.C : 1;
+  const int raw_len = p.transposed && runs == 1 ? p.C * run : run;  // elements of a run of memory
+  auto raw_weights = [&]() {
+    const uint16_t* const src = p.wraw + (size_t)mt * MT * taps_m * (p.transposed ? 1 : p.C);
+    typedef __attribute__((address_space(3))) unsigned char* lds_bytes;
+    const uint32_t lds_at = (uint32_t)(uintptr_t)(lds_bytes)lds_in;
+    const int per = raw_len / 8, pieces = runs * per;  // whole 16-byte pieces (with several runs a run is whole pieces: see the host)
+    for (int i = __builtin_amdgcn_readfirstlane(wave * 64); i < pieces; i += THREADS) {
+      const int at = min(i + lane, pieces - 1), r = runs == 1 ? 0 : at / per;
+      const uint32_t off = 2u * (uint32_t)r * (uint32_t)(p.M * taps_m) + 16u * (uint32_t)(at - r * per);
+      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(src), "s"(lds_at + (uint32_t)i * 16u) : "memory");
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (raw_len % 8 != 0) {  // the last few elements, which share their piece with what lies behind the tensor
+      if (tid < raw_len % 8) reinterpret_cast<uint16_t*>(lds_in)[per * 8 + tid] = src[per * 8 + tid];
+      __syncthreads();
+    }
+  };
+  auto arrange_weights = [&]() {
+    const uint16_t* const raw = reinterpret_cast<const uint16_t*>(lds_in);
+    const int octs = p.wc16 * 2;
+    for (int q = tid; q < octs * MT; q += THREADS) {
+      // Lanes next to each other read from different banks: forward a channel's weights may lie a multiple of the banks apart, so
+      // that eight of them and eight octets go together
+      const int hi = p.transposed ? q / MT : (q >> 3) / octs;
+      const int m = p.transposed ? q % MT : hi * 8 + (q & 7), o = p.transposed ? hi : (q >> 3) - hi * octs;
+      const int kd = o * 8 / p.Cp, c0 = o * 8 - kd * p.Cp;
+      const int first = p.transposed ? (c0 * left_m + m) * taps_m + (p.KD - 1 - kd) * TAPS : (m * p.C + c0) * taps_m + kd * TAPS;
+      const int step = p.transposed ? left_m * taps_m : taps_m;
+      const int have = m < left_m ? min(p.C - c0, 8) : 0;  // channels of the octet that exist
+      u32x4 v[WTAPS];
+#pragma unroll
+      for (int t = 0; t < WTAPS; ++t) v[t] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint16_t* const w = raw + (j < have ? first + j * step : 0);
+        const uint32_t keep = j < have ? 0xffffu : 0u;
+#pragma unroll
+        for (int t = 0; t < WTAPS; ++t) {
+          uint32_t bits;
+          if (MODE == STRIDED_DGRAD) bits = phase_has(blockIdx.y & 1, t) ? w[phase_tap(blockIdx.y & 1, t)] : 0u;
+          else bits = w[t];
+          v[t][j / 2] |= (bits & keep) << (16 * (j & 1));
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < WTAPS; ++t) {
+        const int tap = MODE != STRIDED_DGRAD && p.transposed ? TAPS - 1 - t : t;
+        lds_w[((size_t)tap * octs + o) * MT + m] = v[t];
+      }
+    }
+    __syncthreads();
   };
   auto transfers_landed = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
   if (tid < MT)
@@ -1478,7 +1542,12 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   int buf = 0;
   cursor_enter(0);
   issue_stage();
-  if (p.ngroups == 1) load_weights(0);
+  if (p.wraw != nullptr) {
+    raw_weights();
+    arrange_weights();
+  } else if (p.ngroups == 1) {
+    load_weights(0);
+  }
   store_stage(0, 0);
   transfers_landed();
   if (stages > 1) issue_stage();
@@ -1733,6 +1802,15 @@ Tiling tiling_of(const Launch& L, int Hout, int Wout, bool wide_rows, bool even,
   return best;
 }
 
+// Whether a workgroup's share of the weights can be fetched in whole 16-byte pieces (all but the last few elements of a tensor)
+// and fits the stage buffers, filled 64 pieces at a time.
+bool raw_weights_fit(const Launch& L, int MT) {
+  if ((reinterpret_cast<uintptr_t>(L.w) & 15) != 0) return false;
+  const long long taps_m = (long long)L.KD * TAPS, tile = std::min(MT, L.M);
+  if (L.transposed && L.M > MT && L.M % 8 != 0) return false;  // runs of a tile's channels, one for each contraction channel
+  return (tile * L.C * taps_m + 511) / 512 * 1024 <= 2 * (long long)STAGE_BYTES;
+}
+
 int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const char* who) {
   const SplitSpec sp = split_spec(L.split);
   const bool joined = joined_blocks(L.split, L.KD, L.C);
@@ -1761,6 +1839,8 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
   const size_t total_w = lay.prep_bytes / 2;
   JG_REQUIRE(total_w < (1ull << 31), "%s: weight tensor too large", who);
   const uint16_t* x16 = static_cast<const uint16_t*>(L.x);
+  // Each workgroup puts its weights in order itself where they are 16-bit, stay in LDS and pass through the stage buffers: see arrange_weights
+  const bool arranged = !L.split && lay.ngroups == 1 && raw_weights_fit(L, MT);
   if (L.split) {
     const unsigned wblocks = (unsigned)((total_w + 255) / 256);
     uint16_t* xs = reinterpret_cast<uint16_t*>(static_cast<char*>(ws) + (lay.prep_bytes + 255) / 256 * 256);
@@ -1779,7 +1859,7 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
     JG_CHECK_LAUNCH(who);
     if (rc) return rc;
     x16 = xs;
-  } else {
+  } else if (!arranged) {
     prep_weights_kernel<<<(unsigned)((total_w + 255) / 256), 256, 0, s>>>(wprep, static_cast<const uint16_t*>(L.w), L.M,
                                                                            L.C, pad16(L.C), L.KD, MT, lay.mtiles,
                                                                            lay.wc16, lay.ngroups, L.transposed);
@@ -1789,6 +1869,8 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
   FwdParams p;
   p.x_end = reinterpret_cast<const char*>(x16) + 2 * x_elements * copies;
   p.x = x16; p.wprep = reinterpret_cast<const u32x4*>(wprep);
+  p.wraw = arranged ? static_cast<const uint16_t*>(L.w) : nullptr;
+  p.transposed = L.transposed;
   p.bias = static_cast<const uint16_t*>(L.bias); p.y = static_cast<uint16_t*>(L.y);
   p.N = L.N; p.C = C; p.M = L.M; p.KD = L.KD;
   p.Cp = pad16(C);

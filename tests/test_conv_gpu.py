@@ -845,7 +845,7 @@ def test_rows_and_columns_beside_the_tile_grid(case, dtype, dev):
     # batch, c_in, c_out, size, stride: tiles of 64 produced channels (launches that fill the chip) and, with fewer images, of 32; whole
     # 16-byte rows and others, channels that end inside a tile, more contraction steps than LDS holds weights for
     (600, 16, 64, (16, 64), 1), (40, 16, 64, (16, 64), 1), (600, 7, 50, (9, 33), 1), (40, 7, 50, (9, 33), 1), (300, 80, 64, (5, 40), 1), (3, 80, 128, (5, 40), 1),
-    (600, 16, 64, (16, 64), 2), (40, 16, 64, (16, 64), 2), (600, 9, 60, (11, 35), 2), (30, 70, 60, (11, 35), 2),
+    (600, 16, 64, (16, 64), 2), (40, 16, 64, (16, 64), 2), (600, 9, 60, (11, 35), 2), (30, 70, 60, (11, 35), 2), (3, 88, 24, (10, 30), 2), (3, 5, 9, (10, 30), 1),
 ], ids=str)
 def test_tiles_of_64_and_of_32_channels_exactly(case, dtype, dev):
     """Whole numbers, as in test_strided_3x3_layers_exactly."""
@@ -857,6 +857,10 @@ def test_tiles_of_64_and_of_32_channels_exactly(case, dtype, dev):
     want = torch.nn.functional.conv2d(x, w, b, stride=stride, padding=1)  # sums below 2^24: exact in fp32
     y = jc.conv_nd(x.to(dtype).to(dev), w.to(dtype).to(dev), b.to(dtype).to(dev), stride=stride, padding=1)
     assert torch.equal(y.cpu(), want.to(dtype))
+    # the input gradient, whose workgroups put the same weights in another order: channel by channel, where that is whole 16-byte pieces
+    g = torch.randint(-1, 2, want.shape, generator=gen).float()
+    gx = jc.conv_nd_input(x.shape, w.to(dtype).to(dev), g.to(dtype).to(dev), stride=stride, padding=1)
+    assert torch.equal(gx.cpu(), torch.nn.grad.conv2d_input(x.shape, w, g, stride=stride, padding=1).to(dtype))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
