@@ -22,12 +22,6 @@ int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
                          const void* const* k, const void* const* v, int nchunks, const void* out, const float* lse,
                          long long batch, int sq, int sk, float scale, void* ws, hipStream_t s);
 bool attn_wide_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias);
-int attn_wide_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v, int nchunks,
-                         long long batch, int sq, int sk, int d, int dtype, float scale, float* out_acc, float* lse_acc,
-                         hipStream_t s);
-int attn_wide_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q,
-                         const void* const* k, const void* const* v, int nchunks, const void* out, const float* lse,
-                         long long batch, int sq, int sk, int d, int dtype, float scale, void* ws, hipStream_t s);
 bool attn_f32_mfma_fwd_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias);
 int attn_f32_mfma_fwd(void* out, float* lse, const void* q, const void* k, const void* v, long long batch, int sq,
                       int sk, int d, float scale, float* out_acc, float* lse_acc, hipStream_t s);

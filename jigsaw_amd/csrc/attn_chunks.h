@@ -80,6 +80,25 @@ __device__ __forceinline__ void parts8(const float* v, bf16x8_t (&part)[3]) {
   for (int t = 0; t < 3; ++t) part[t] = __builtin_bit_cast(bf16x8_t, w[t]);
 }
 
+// Wavefronts of 32 rows each that share a tile of the streamed side in the kernels of attn_wide.hip: four, or as many fewer as it takes
+// to give every compute unit a workgroup. A tile takes 1.3 to 2.5 us of latency whatever else runs there (fetch, scores, exponentials,
+// products, one after the other), so that 48 workgroups of 128 rows left the chip idle for as long as a full one; with 64 or 32 rows they
+// are two or four times as many, and what their fewer rows leave free takes more tiles at once (four to eight groups a workgroup). Forward / backward,
+// us, before -> with it: 1 x 8 heads x 512 x 4 chunks, head size 128 47 / 84 -> 32 / 59, fp16 64 29 / 46 -> 17 / 30, 8 chunks at 32 39 / 59 -> 19 / 32;
+// 4 x 1006 x 5, 80 92 / 124 -> 53 / 83; 2 x 197 x 5, fp16 96 47 / 41 -> 24 / 26. Forced, where 128 rows have a workgroup for every second
+// compute unit or more: 60 x 529 x 4, fp16 96 94 / 190 -> 125 / 209 (64 rows); at head size 32, whose workgroups fit a compute unit several times,
+// up to two of 64 rows each still gain: 28 x 931 x 7 84 / 156 -> 78 / 152, 14 x 1442 x 5 87 / 153 -> 77 / 139.
+inline int attn_width(long long rows, long long batch, int columns) {
+  if (cdiv(rows, 32) * batch <= cu_count()) return 1;
+  return cdiv(rows, 64) * batch <= (columns == 32 ? 2 : 1) * cu_count() ? 2 : 4;
+}
+// (attn_wide.hip; dk, dv NULL: dQ and delta only)
+int attn_wide_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v, int nchunks,
+                         long long batch, int sq, int sk, int d, int dtype, float scale, float* out_acc, float* lse_acc, hipStream_t s);
+int attn_wide_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q, const void* const* k,
+                         const void* const* v, int nchunks, const void* out, const float* lse, long long batch, int sq,
+                         int sk, int d, int dtype, float scale, void* ws, hipStream_t s);
+
 // Workgroup -> (batch entry, chunk, row block) of a grid (row blocks, batch entries, chunks). Consecutive
 // workgroup ids go to the 8 XCDs in turn; each XCD is given a contiguous range of the flat order (batch entry,
 // chunk, block), so the workgroups that stream the same K / V (or Q / dO) share one L2 instead of every L2

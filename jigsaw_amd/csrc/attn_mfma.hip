@@ -569,8 +569,13 @@ bool attn_mfma_fwd_supported(long long batch, int sq, int sk, int d, int dtype, 
   return dtype == JG_BF16 && !has_bias && d == D && sq > 0 && sk > 0 && sk <= ATTN_MAX_KEYS && batch > 0 && batch <= 65535;
 }
 
+// Launches of few workgroups of 128 queries go to the kernels that split them further (attn_width; the same keys keep their
+// probabilities in fp32 there): 1 x 8 heads x 512 x 4 chunks 24.7 -> 16.6 us, 1 x 8 x 1024 x 8 72 -> 53, 24 x 95 x 3 15.2 -> 11.9, 16 x 1000 x 2
+// 28.6 -> 24.6, 8 x 2000 x 2 45 -> 42.
 int attn_mfma_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v, int nchunks,
                          long long batch, int sq, int sk, float scale, float* out_acc, float* lse_acc, hipStream_t s) {
+  if (attn_width(sq, batch, D) < 4)
+    return attn_wide_fwd_chunks(out, lse, q, k, v, nchunks, batch, sq, sk, D, JG_BF16, scale, out_acc, lse_acc, s);
   FwdArgs a;
   a.q = static_cast<const uint16_t*>(q);
   a.out = static_cast<uint16_t*>(out);

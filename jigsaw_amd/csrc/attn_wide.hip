@@ -8,10 +8,11 @@
 //   widths         kernels of 32, 64, 96 and 128 columns (D); a smaller head is staged with zeros in
 //                  the columns it does not have. Rows past the end of a tensor are staged as zeros
 //                  too; keys past the end get the score -inf, queries past the end the lse +inf.
-//   groups         a workgroup is KS groups of four wavefronts. A group walks every KS-th tile of
+//   groups         a workgroup is KS groups of W wavefronts. A group walks every KS-th tile of
 //                  the streamed side with a stage of its own, and the groups' sums are combined
 //                  through LDS at the end: where a launch has fewer workgroups than the chip has
-//                  CUs, more wavefronts share the rows of one (see split_of on the host side).
+//                  CUs, more wavefronts share the rows of one (see two_groups on the host side), and
+//                  where it has fewer than half, workgroups have 64 or 32 rows (attn_width).
 //
 // Forward + backward of a ring, before (lengths and head size padded on the host, one launch and one merge per
 // chunk) and in one launch each: 4 heads x 128 x 2 chunks of 128 keys, head size 32: 402 -> 48 us (host time); 12 heads x 869 x 869,
@@ -60,8 +61,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int WAVES = 4, GROUP = WAVES * 64;  // wavefronts and threads of a group
-constexpr int BQ = 32 * WAVES;  // rows (queries or keys) of a workgroup, 32 per wavefront of a group
+// W: wavefronts of a group. A workgroup has 32 W rows (queries or keys), 32 per wavefront of a group, a group 64 W threads.
 constexpr int BT = 32;          // rows of a streamed tile
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float NO_SCORE = -1.0e30f;  // running maximum before the first key: finite, so that a group without a key weighs 0
@@ -77,32 +77,32 @@ struct Geo {
   __device__ static __forceinline__ int swizzle(int r) { return ((r >> 2) & 3) | (D == 64 ? ((r >> 1) & 1) << 2 : (D == 128 ? (r & 3) << 2 : 0)); }
   static constexpr int RV = D == 64 ? 4 : (D == 128 ? 8 : 2), TV = RV / 2;  // pieces, and blocks of 32 columns, whose swizzles differ
   static constexpr int CHUNKS = BT * D / 8;  // 16-byte pieces of a tile
-  static constexpr int PER = (CHUNKS + GROUP - 1) / GROUP;
 };
 
-template <int D>
+template <int D, int W>
 struct TileRegs {
-  u32x4 v[Geo<D>::PER];
+  static constexpr int GROUP = W * 64, PER = (Geo<D>::CHUNKS + GROUP - 1) / GROUP;
+  u32x4 v[PER];
   int rows;
 };
 
 // 32 rows of a row-major matrix of row length d <= D to registers; rows from `rows` on and columns from d on become zero on their way to LDS.
 // They are read from the last row and piece there is: a load under a condition is waited for where the paths meet, on the spot (24 heads x
 // 739 x 5 chunks, head size 32: forward 63 -> 48 us, dQ 54 -> 46). tid: thread of the group; at least one row lies before `rows`.
-template <int D>
-__device__ __forceinline__ void tile_fetch(TileRegs<D>& r, const uint16_t* src, int tid, int rows, int d) {
+template <int D, int W>
+__device__ __forceinline__ void tile_fetch(TileRegs<D, W>& r, const uint16_t* src, int tid, int rows, int d) {
   r.rows = rows;
 #pragma unroll
-  for (int i = 0; i < Geo<D>::PER; ++i) {
-    const int c = min(tid + i * GROUP, Geo<D>::CHUNKS - 1);
+  for (int i = 0; i < TileRegs<D, W>::PER; ++i) {
+    const int c = min(tid + i * (W * 64), Geo<D>::CHUNKS - 1);
     r.v[i] = *reinterpret_cast<const u32x4*>(src + min(c / (D / 8), rows - 1) * d + min(c % (D / 8) * 8, d - 8));
   }
 }
-template <int D>
-__device__ __forceinline__ void tile_store(const TileRegs<D>& r, unsigned char* dst, int tid, int d) {
+template <int D, int W>
+__device__ __forceinline__ void tile_store(const TileRegs<D, W>& r, unsigned char* dst, int tid, int d) {
 #pragma unroll
-  for (int i = 0; i < Geo<D>::PER; ++i) {
-    const int c = tid + i * GROUP;
+  for (int i = 0; i < TileRegs<D, W>::PER; ++i) {
+    const int c = tid + i * (W * 64);
     if (c < Geo<D>::CHUNKS) {
       const int row = c / (D / 8), piece = c % (D / 8);
       const bool there = row < r.rows && piece * 8 < d;
@@ -284,18 +284,18 @@ struct Args {
 // What it costs, forward / backward of 64 heads x 100 queries x 8 chunks of 100 keys, rounded -> not: bf16, head size 64
 // 33 / 52 -> 34 / 58 us, 96 34 / 62 -> 40 / 78, 128 (127 keys) 35 / 86 -> 49 / 102; fp16, whose operands go in as two parts, 64
 // 34 / 52 -> 45 / 79. The one-thread-per-row kernels, which these chunks ran before, took 1107 / 2418 us at bf16 64, eight launches each way.
-template <int D, bool F16, int KS, bool EXACT>
-__global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, Args p) {
+template <int D, bool F16, int W, int KS, bool EXACT>
+__global__ __launch_bounds__(64 * W * KS) void attn_wide_fwd_kernel(ChunkTable, Args p) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
   constexpr int BUF = 2 * G::TILE;  // K tile, V tile
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int tid = threadIdx.x % GROUP, ks = threadIdx.x / GROUP;
+  const int tid = threadIdx.x % (64 * W), ks = threadIdx.x / (64 * W);
   const int lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kg = lane >> 5;
   const BlockOf wg = block_of();
   const long long bh = wg.bh;
-  const int qi = wg.blk * BQ + wave * 32 + ln;
+  const int qi = wg.blk * (32 * W) + wave * 32 + ln;
   const bool live = qi < p.sq;
   const uint16_t* qrow = p.q + (bh * p.sq + (live ? qi : p.sq - 1)) * p.d;
   const long long chunk_off = bh * p.sk * p.d;
@@ -318,20 +318,20 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
     const bool exact = EXACT && pass == 1;
     const int lo = exact ? p.exact_from : 0, hi = EXACT && !exact ? p.exact_from : p.sk;
     if (EXACT && lo == hi) continue;
-    TileRegs<D> rk, rv;
+    TileRegs<D, W> rk, rv;
     Stream<KS> load(lo, hi, ks), soft(lo, hi, ks);
     const int ntiles = load.steps * p.nchunks;
     auto fetch = [&]() {
       const uint16_t* kb = reinterpret_cast<const uint16_t*>(chunk_entry(0, load.chunk)) + chunk_off;
       const uint16_t* vb = reinterpret_cast<const uint16_t*>(chunk_entry(1, load.chunk)) + chunk_off;
       const long long at = (long long)load.first_row() * p.d;
-      tile_fetch<D>(rk, kb + at, tid, load.rows_left(), p.d);
-      tile_fetch<D>(rv, vb + at, tid, load.rows_left(), p.d);
+      tile_fetch<D, W>(rk, kb + at, tid, load.rows_left(), p.d);
+      tile_fetch<D, W>(rv, vb + at, tid, load.rows_left(), p.d);
       load.next();
     };
     auto store = [&](int buf) {
-      tile_store<D>(rk, lds + buf * BUF, tid, p.d);
-      tile_store<D>(rv, lds + buf * BUF + G::TILE, tid, p.d);
+      tile_store<D, W>(rk, lds + buf * BUF, tid, p.d);
+      tile_store<D, W>(rv, lds + buf * BUF + G::TILE, tid, p.d);
     };
     fetch();
     store(0);
@@ -407,11 +407,11 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
   if constexpr (KS > 1) {
     // the groups hand over to the one below them, halving their number each time
     constexpr int XO = (16 * G::NB + 2) * 64;  // floats of a wavefront (in the stages' place, see launch_fwd)
-    float* xo = reinterpret_cast<float*>(smem) + ((ks % (KS / 2)) * WAVES + wave) * XO + lane;
+    float* xo = reinterpret_cast<float*>(smem) + ((ks % (KS / 2)) * W + wave) * XO + lane;
 #pragma unroll
     for (int half = KS / 2; half >= 1; half >>= 1) {
       if (ks >= half && ks < 2 * half) {
-        float* to = reinterpret_cast<float*>(smem) + ((ks - half) * WAVES + wave) * XO + lane;
+        float* to = reinterpret_cast<float*>(smem) + ((ks - half) * W + wave) * XO + lane;
 #pragma unroll
         for (int nb = 0; nb < G::NB; ++nb)
 #pragma unroll
@@ -472,21 +472,45 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_fwd_kernel(ChunkTable, A
     }
 }
 
+// The groups' sums to group 0: each hands over to the one below it, halving their number each time (in the stages' place, which a
+// barrier has closed).
+template <int NB, int W, int KS>
+__device__ __forceinline__ void hand_over(float* lds, int ks, int wave, int lane, f32x16 (&sum)[NB]) {
+#pragma unroll
+  for (int half = KS / 2; half >= 1; half >>= 1) {
+    float* const at = lds + ((ks % half) * W + wave) * (16 * NB * 64) + lane;
+    if (ks >= half && ks < 2 * half) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) at[(nb * 16 + i) * 64] = sum[nb][i];
+    }
+    __syncthreads();
+    if (ks < half) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sum[nb][i] += at[(nb * 16 + i) * 64];
+    }
+    __syncthreads();
+  }
+}
+
 // ------------------------------------------------------------------- dQ (and delta)
 // EXACT (here and in the dK/dV kernel): dS and the probabilities are not rounded (chunks of fewer than EXACT_KEYS keys).
-template <int D, bool F16, int KS, bool EXACT>
-__global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Args p) {
+template <int D, bool F16, int W, int KS, bool EXACT>
+__global__ __launch_bounds__(64 * W * KS) void attn_wide_dq_kernel(ChunkTable, Args p) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
   constexpr int BUF = 2 * G::TILE;  // K tile, V tile
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int tid = threadIdx.x % GROUP, ks = threadIdx.x / GROUP;
+  const int tid = threadIdx.x % (64 * W), ks = threadIdx.x / (64 * W);
   const int lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kg = lane >> 5;
   const BlockOf wg = block_of();
   const long long bh = wg.bh;
-  const bool live = wg.blk * BQ + wave * 32 + ln < p.sq;
-  const int qi = live ? wg.blk * BQ + wave * 32 + ln : p.sq - 1;
+  const bool live = wg.blk * (32 * W) + wave * 32 + ln < p.sq;
+  const int qi = live ? wg.blk * (32 * W) + wave * 32 + ln : p.sq - 1;
   const long long qoff = (bh * p.sq + qi) * p.d;
   const long long chunk_off = bh * p.sk * p.d;
   const float c2 = p.scale * LOG2E;
@@ -512,21 +536,21 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
 #pragma unroll
   for (int nb = 0; nb < G::NB; ++nb) dq[nb] = zero16();
 
-  TileRegs<D> rk, rv;
+  TileRegs<D, W> rk, rv;
   Stream<KS> load(0, p.sk, ks), soft(0, p.sk, ks);
   const int ntiles = load.steps * p.nchunks;
   auto fetch = [&]() {
     const long long at = chunk_off + (long long)load.first_row() * p.d;
     const uint16_t* kb = reinterpret_cast<const uint16_t*>(chunk_entry(0, load.chunk)) + at;
     const uint16_t* vb = reinterpret_cast<const uint16_t*>(chunk_entry(1, load.chunk)) + at;
-    tile_fetch<D>(rk, kb, tid, load.rows_left(), p.d);
-    tile_fetch<D>(rv, vb, tid, load.rows_left(), p.d);
+    tile_fetch<D, W>(rk, kb, tid, load.rows_left(), p.d);
+    tile_fetch<D, W>(rv, vb, tid, load.rows_left(), p.d);
     load.next();
   };
   auto store = [&](int buf) {
     unsigned char* at = lds + buf * BUF;
-    tile_store<D>(rk, at, tid, p.d);
-    tile_store<D>(rv, at + G::TILE, tid, p.d);
+    tile_store<D, W>(rk, at, tid, p.d);
+    tile_store<D, W>(rv, at + G::TILE, tid, p.d);
   };
   fetch();
   store(0);
@@ -576,20 +600,8 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
   }
   if (t < ntiles) tile(t, 0);
   if constexpr (KS > 1) {
-    static_assert(KS == 2, "one hand-over");
-    float* xo = reinterpret_cast<float*>(smem) + wave * 16 * G::NB * 64 + lane;
-    if (ks == 1) {
-#pragma unroll
-      for (int nb = 0; nb < G::NB; ++nb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) xo[(nb * 16 + i) * 64] = dq[nb][i];
-    }
-    __syncthreads();
-    if (ks == 1) return;
-#pragma unroll
-    for (int nb = 0; nb < G::NB; ++nb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) dq[nb][i] += xo[(nb * 16 + i) * 64];
+    hand_over<G::NB, W, KS>(reinterpret_cast<float*>(smem), ks, wave, lane, dq);
+    if (ks != 0) return;
   }
   if (!live) return;
   uint16_t* row = p.dq + qoff;
@@ -610,21 +622,21 @@ __global__ __launch_bounds__(GROUP * KS) void attn_wide_dq_kernel(ChunkTable, Ar
 // that way), so head sizes above 96 run the kernel twice: MODE 1 forms dV only (from P), MODE 2 dK only
 // (from dS), each with one accumulator and two workgroups per CU; the scores are computed in both.
 // A launch with no more workgroups than CUs gains nothing from that and keeps the single pass.
-template <int D, bool F16, int MODE, int KS, bool EXACT>
-__global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 : 1) void attn_wide_dkv_kernel(ChunkTable, Args p) {
+template <int D, bool F16, int MODE, int W, int KS, bool EXACT>
+__global__ __launch_bounds__(64 * W * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 : 1) void attn_wide_dkv_kernel(ChunkTable, Args p) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
   constexpr bool DV = MODE != 2, DK = MODE != 1;
   constexpr int STATS = 2 * BT * 4;                           // lse * log2(e) and delta of the tile's queries
   constexpr int BUF = 2 * G::TILE + STATS;                    // Q tile, dO tile, stats
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int tid = threadIdx.x % GROUP, ks = threadIdx.x / GROUP;
+  const int tid = threadIdx.x % (64 * W), ks = threadIdx.x / (64 * W);
   const int lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kg = lane >> 5;
   const BlockOf wg = block_of();
   const long long bh = wg.bh;
-  const bool live = wg.blk * BQ + wave * 32 + ln < p.sk;
-  const long long koff = (bh * p.sk + (live ? wg.blk * BQ + wave * 32 + ln : p.sk - 1)) * p.d;
+  const bool live = wg.blk * (32 * W) + wave * 32 + ln < p.sk;
+  const long long koff = (bh * p.sk + (live ? wg.blk * (32 * W) + wave * 32 + ln : p.sk - 1)) * p.d;
   const uint16_t* qb = p.q + bh * p.sq * p.d;
   const uint16_t* gb = p.dout + bh * p.sq * p.d;
   const float* lb = p.lse_in + bh * p.sq;
@@ -650,7 +662,7 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
     if (DV) dv[nb] = zero16();
   }
 
-  TileRegs<D> rq, rg;
+  TileRegs<D, W> rq, rg;
   float st = 0.0f;  // one statistic per thread of the group's first wavefront: lse2 (lanes 0-31) or delta (32-63)
   int st_rows = 0;  // rows of the tile it belongs to
   Stream<KS> load(0, p.sq, ks);
@@ -658,8 +670,8 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
   auto fetch = [&]() {
     const long long at = (long long)load.first_row() * p.d;
     const int rows = load.rows_left();
-    tile_fetch<D>(rq, qb + at, tid, rows, p.d);
-    tile_fetch<D>(rg, gb + at, tid, rows, p.d);
+    tile_fetch<D, W>(rq, qb + at, tid, rows, p.d);
+    tile_fetch<D, W>(rg, gb + at, tid, rows, p.d);
     if (tid < 2 * BT) {
       const float* src = tid < BT ? lb : db;  // every lane loads; the factor is applied when stored
       st = src[min(load.first_row() + (tid & (BT - 1)), p.sq - 1)];
@@ -669,8 +681,8 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
   };
   auto store = [&](int buf) {
     unsigned char* base = lds + buf * BUF;
-    tile_store<D>(rq, base, tid, p.d);
-    tile_store<D>(rg, base + G::TILE, tid, p.d);
+    tile_store<D, W>(rq, base, tid, p.d);
+    tile_store<D, W>(rg, base + G::TILE, tid, p.d);
     if (tid < 2 * BT) {
       float v = tid < BT ? st * LOG2E : st;
       if ((tid & (BT - 1)) >= st_rows) v = tid < BT ? INFINITY : 0.0f;  // a query past the end: probability 0
@@ -752,26 +764,10 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
     if (t < ntiles) tile(t, 0);
   }
   if constexpr (KS > 1) {
-    static_assert(KS == 2 && MODE == 0, "one hand-over of both sums");
-    float* xo = reinterpret_cast<float*>(smem) + wave * 32 * G::NB * 64 + lane;
-    if (ks == 1) {
-#pragma unroll
-      for (int nb = 0; nb < G::NB; ++nb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          xo[(nb * 16 + i) * 64] = dk[nb][i];
-          xo[((G::NB + nb) * 16 + i) * 64] = dv[nb][i];
-        }
-    }
-    __syncthreads();
-    if (ks == 1) return;
-#pragma unroll
-    for (int nb = 0; nb < G::NB; ++nb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        dk[nb][i] += xo[(nb * 16 + i) * 64];
-        dv[nb][i] += xo[((G::NB + nb) * 16 + i) * 64];
-      }
+    static_assert(MODE == 0, "hand-over of both sums");
+    hand_over<G::NB, W, KS>(reinterpret_cast<float*>(smem), ks, wave, lane, dk);
+    hand_over<G::NB, W, KS>(reinterpret_cast<float*>(smem), ks, wave, lane, dv);
+    if (ks != 0) return;
   }
   if (!live) return;
   uint16_t* krow = reinterpret_cast<uint16_t*>(const_cast<char*>(chunk_entry(2, wg.chunk))) + koff;
@@ -791,13 +787,9 @@ __global__ __launch_bounds__(GROUP * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 :
     }
 }
 
-// Groups per workgroup. A launch that leaves CUs without a workgroup splits the streamed side over more wavefronts
-// of one: up to 4 groups where the registers of 16 wavefronts hold the state (forward, D <= 64), else 2.
-int split_of(long long workgroups, int most) {
-  int ks = 1;
-  while (ks < most && workgroups * ks < jg::cu_count()) ks *= 2;
-  return ks;
-}
+// Workgroups of 128 rows (attn_width: half of the CUs and more have one; at head size 32 all of them, twice): where some CU has none, two
+// groups share the streamed side.
+bool two_groups(long long workgroups) { return workgroups < jg::cu_count(); }
 
 // `args` in a launch of `kernel` that needs more LDS than the default limit
 template <typename K>
@@ -810,45 +802,77 @@ int launch(K kernel, dim3 grid, int threads, int lds, const ChunkTable& tab, con
   return JG_OK;
 }
 
+typedef std::integral_constant<int, 1> One;
+typedef std::integral_constant<int, 2> Two;
+typedef std::integral_constant<int, 4> Four;
+template <int D>
+using Most = std::integral_constant<int, D <= 64 ? 8 : 4>;  // groups of one wavefront each whose stages LDS holds
+
 template <int D, bool F16, bool EXACT>
 int launch_fwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
   typedef Geo<D> G;
-  constexpr int LDS = 2 * 2 * G::TILE, SUMS = WAVES * (16 * G::NB + 2) * 64 * 4;  // stages; what a group hands over
-  auto lds = [](int ks) { return std::max(ks * LDS, ks / 2 * SUMS); };
-  const dim3 grid((unsigned)jg::cdiv(a.sq, BQ), (unsigned)batch, 1);
-  const char* who = "jg_attn_fwd(wide)";
-  const int ks = split_of((long long)grid.x * batch, D <= 64 ? 4 : 2);
-  if constexpr (D <= 64)
-    if (ks == 4) return launch(&attn_wide_fwd_kernel<D, F16, 4, EXACT>, grid, 4 * GROUP, lds(4), tab, a, s, who);
-  if (ks == 2) return launch(&attn_wide_fwd_kernel<D, F16, 2, EXACT>, grid, 2 * GROUP, lds(2), tab, a, s, who);
-  return launch(&attn_wide_fwd_kernel<D, F16, 1, EXACT>, grid, GROUP, LDS, tab, a, s, who);
+  auto go = [&](auto w, auto k) {
+    constexpr int W = decltype(w)::value, KS = decltype(k)::value;
+    constexpr int STAGES = KS * 2 * 2 * G::TILE, SUMS = KS / 2 * W * (16 * G::NB + 2) * 64 * 4;  // stages; what the groups hand over
+    static_assert(STAGES <= 160 * 1024 && SUMS <= 160 * 1024, "fits LDS");
+    return launch(&attn_wide_fwd_kernel<D, F16, W, KS, EXACT>, dim3((unsigned)jg::cdiv(a.sq, 32 * W), (unsigned)batch, 1), 64 * W * KS,
+                  std::max(STAGES, SUMS), tab, a, s, "jg_attn_fwd(wide)");
+  };
+  switch (jg::attn_width(a.sq, batch, D)) {
+    case 1: return go(One{}, Most<D>{});
+    case 2: return go(Two{}, Four{});
+  }
+  if constexpr (D > 32)
+    if (two_groups(jg::cdiv(a.sq, 128) * batch)) return go(Four{}, Two{});
+  return go(Four{}, One{});
 }
 
 template <int D, bool F16, bool EXACT>
-int launch_bwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
+int launch_dq(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
   typedef Geo<D> G;
-  constexpr int DQ_LDS = 2 * 2 * G::TILE, DKV_LDS = 2 * (2 * G::TILE + 2 * BT * 4);  // stages
-  constexpr int SUMS = WAVES * 16 * G::NB * 64 * 4;                                  // what a group hands over of each
-  const dim3 dq_grid((unsigned)jg::cdiv(a.sq, BQ), (unsigned)batch, 1);
-  const dim3 dkv_grid((unsigned)jg::cdiv(a.sk, BQ), (unsigned)batch, (unsigned)a.nchunks);
-  const long long dkv_workgroups = (long long)dkv_grid.x * batch * a.nchunks;
-  const char* who = "jg_attn_bwd(wide, dq)";
-  int rc = split_of((long long)dq_grid.x * batch, 2) == 2
-               ? launch(&attn_wide_dq_kernel<D, F16, 2, EXACT>, dq_grid, 2 * GROUP, std::max(2 * DQ_LDS, SUMS), tab, a, s, who)
-               : launch(&attn_wide_dq_kernel<D, F16, 1, EXACT>, dq_grid, GROUP, DQ_LDS, tab, a, s, who);
-  if (rc != JG_OK) return rc;
-  who = "jg_attn_bwd(wide, dkv)";
+  auto go = [&](auto w, auto k) {
+    constexpr int W = decltype(w)::value, KS = decltype(k)::value;
+    constexpr int STAGES = KS * 2 * 2 * G::TILE, SUMS = KS / 2 * W * 16 * G::NB * 64 * 4;
+    static_assert(STAGES <= 160 * 1024 && SUMS <= 160 * 1024, "fits LDS");
+    return launch(&attn_wide_dq_kernel<D, F16, W, KS, EXACT>, dim3((unsigned)jg::cdiv(a.sq, 32 * W), (unsigned)batch, 1), 64 * W * KS,
+                  std::max(STAGES, SUMS), tab, a, s, "jg_attn_bwd(wide, dq)");
+  };
+  switch (jg::attn_width(a.sq, batch, D)) {
+    case 1: return go(One{}, Most<D>{});
+    case 2: return go(Two{}, Four{});
+  }
+  if constexpr (D > 32)
+    if (two_groups(jg::cdiv(a.sq, 128) * batch)) return go(Four{}, Two{});
+  return go(Four{}, One{});
+}
+
+template <int D, bool F16, bool EXACT>
+int launch_dkv(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
+  typedef Geo<D> G;
+  auto go = [&](auto mode, auto w, auto k) {
+    constexpr int W = decltype(w)::value, KS = decltype(k)::value;
+    constexpr int STAGES = KS * 2 * (2 * G::TILE + 2 * BT * 4), SUMS = KS / 2 * W * 16 * G::NB * 64 * 4;
+    static_assert(STAGES <= 160 * 1024 && SUMS <= 160 * 1024, "fits LDS");
+    return launch(&attn_wide_dkv_kernel<D, F16, decltype(mode)::value, W, KS, EXACT>,
+                  dim3((unsigned)jg::cdiv(a.sk, 32 * W), (unsigned)batch, (unsigned)a.nchunks), 64 * W * KS, std::max(STAGES, SUMS), tab, a, s,
+                  "jg_attn_bwd(wide, dkv)");
+  };
+  typedef std::integral_constant<int, 0> Both;
+  const long long workgroups = jg::cdiv(a.sk, 128) * batch * a.nchunks;
+  switch (jg::attn_width(a.sk, batch * a.nchunks, D)) {  // (four wavefronts: a head of 128 then has the registers for both sums)
+    case 1: return go(Both{}, One{}, Four{});
+    case 2: return go(Both{}, Two{}, Two{});
+  }
   // up to head size 96 (64 with EXACT): dK and dV in one pass; above: one pass each when the launch has more workgroups
   // than the chip has CUs, and with EXACT always (register budget, see the kernel)
   if constexpr (D <= (EXACT ? 64 : 96)) {
-    if (split_of(dkv_workgroups, 2) == 2)
-      return launch(&attn_wide_dkv_kernel<D, F16, 0, 2, EXACT>, dkv_grid, 2 * GROUP, std::max(2 * DKV_LDS, 2 * SUMS), tab, a, s, who);
-  } else if (EXACT || dkv_workgroups > jg::cu_count()) {
-    rc = launch(&attn_wide_dkv_kernel<D, F16, 1, 1, EXACT>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
-    if (rc != JG_OK) return rc;
-    return launch(&attn_wide_dkv_kernel<D, F16, 2, 1, EXACT>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
+    if constexpr (D > 32)
+      if (two_groups(workgroups)) return go(Both{}, Four{}, Two{});
+  } else if (EXACT || workgroups > jg::cu_count()) {
+    const int rc = go(One{}, Four{}, One{});
+    return rc != JG_OK ? rc : go(Two{}, Four{}, One{});
   }
-  if constexpr (D <= 64 || !EXACT) return launch(&attn_wide_dkv_kernel<D, F16, 0, 1, EXACT>, dkv_grid, GROUP, DKV_LDS, tab, a, s, who);
+  if constexpr (D <= 64 || !EXACT) return go(Both{}, Four{}, One{});
   return JG_OK;
 }
 
@@ -889,6 +913,7 @@ int attn_wide_fwd_chunks(void* out, float* lse, const void* q, const void* const
   });
 }
 
+// dk, dv NULL: dQ (and delta) only
 int attn_wide_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q, const void* const* k,
                          const void* const* v, int nchunks, const void* out, const float* lse, long long batch, int sq,
                          int sk, int d, int dtype, float scale, void* ws, hipStream_t s) {
@@ -902,7 +927,10 @@ int attn_wide_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
   a.sq = sq; a.sk = sk; a.d = d; a.nchunks = nchunks; a.scale = scale;
   const ChunkTable tab = chunk_table(k, v, dk, dv, nchunks);
   return by_width(d, dtype, [&](auto width, auto f16) {
-    return sk < EXACT_KEYS ? launch_bwd<width(), f16(), true>(tab, a, batch, s) : launch_bwd<width(), f16(), false>(tab, a, batch, s);
+    const bool exact = sk < EXACT_KEYS;
+    const int rc = exact ? launch_dq<width(), f16(), true>(tab, a, batch, s) : launch_dq<width(), f16(), false>(tab, a, batch, s);
+    if (rc != JG_OK || dk == nullptr) return rc;
+    return exact ? launch_dkv<width(), f16(), true>(tab, a, batch, s) : launch_dkv<width(), f16(), false>(tab, a, batch, s);
   });
 }
 

@@ -546,6 +546,16 @@ _STRAYS = {torch.bfloat16: 0.005, torch.float16: 0.02}
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [32, 64, 88, 128])
+@pytest.mark.parametrize("h,sq,sk,P", [
+    # workgroups of 32, 64 and 128 queries and, apart from them, keys; key groups with fewer tiles than others, none at all, one key
+    (2, 33, 40, 2), (3, 65, 300, 1), (60, 150, 70, 3), (70, 65, 290, 1), (100, 130, 140, 2), (140, 130, 64, 1), (300, 70, 33, 1), (5, 64, 1025, 2), (260, 1, 130, 1),
+])
+def test_workgroups_of_every_width(h, sq, sk, P, d, dtype, dev):
+    test_ring_of_any_lengths_in_one_pass(1, h, sq, sk, d, P, dtype, dev)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("h,sq,sk,d,P", [(4, 100, 100, 64, 2), (4, 300, 127, 64, 3), (3, 64, 31, 64, 1), (4, 100, 65, 40, 2), (3, 130, 97, 32, 5),
                                          (3, 130, 97, 96, 2), (3, 200, 127, 128, 2), (300, 130, 100, 80, 1)], ids=str)
 def test_short_key_ranges_keep_probabilities_in_fp32(h, sq, sk, d, P, dtype, dev):
