@@ -325,7 +325,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
     // (with LEAD the window's last dword holds one pixel more than is used; it shares its dword with one that is)
     const bool rows_inside = oh0 + SR <= p.Hout && ih0 >= 0 && ih0 + NEW <= p.Hin && id0 >= 0 && id0 + KD <= p.Din;
     // All that a stage's loads of x and g reach lies inside the tensors, whatever columns the rows have
-    constexpr bool kWhole = !FRAMED && CXB != 3;  // (built where there are registers for it)
+    constexpr bool kWhole = !FRAMED;  // (the framed kernels have no registers for it)
     auto whole = [&]() {
       const char* const x_last = x_org + 2 * ((size_t)(cin_valid - 1) * x_cs + (size_t)(KD - 1) * plane_x + (size_t)(NEW - 1) * p.Win) + 2 * 64 + 16;
       const char* const g_last = g_org + 2 * ((size_t)(cout_valid - 1) * g_cs + (size_t)(SR - 1) * p.Wout) + 2 * SW + 8;
@@ -707,6 +707,11 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
       // (With six multiplying wavefronts, two SIMDs hold a wavefront that only stages; there the
       // split measured slower, and every wavefront stores and loads between its two groups.)
       const bool stage_first = CWAVES == 8 && (wave & 4) != 0;
+      // Both groups' fragments before the first matrix instruction; not in the kernels of a volume that have edges, where the second
+      // group's 28 registers between the two are what the test of `whole` takes (without it a volume whose rows end inside a strip paid for
+      // every stage what the tensor's ends cost): 1 x 30 -> 9 of 38 x 66 x 15 45.1 -> 40.7 us, 2 x 64 -> 64 of 30 x 50 x 20 79.6 -> 74.1,
+      // 2 x 48 -> 8 of 36 x 48 x 76 83.5 -> 80.0.
+      constexpr bool kBothFirst = CWAVES == 8 || ALLIN || FRAMED;
       for (long long st = s_begin; st < s_end; ++st) {
         Frags f0, f1;
         (void)f1;
@@ -716,7 +721,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
         }
         if (wave < CWAVES) {
           read_group(f0, gbuf, base, 0);
-          if (GROUPS == 2) read_group(f1, gbuf, base, 1);
+          if (GROUPS == 2 && kBothFirst) read_group(f1, gbuf, base, 1);
           mfma_group(f0);
           if (GROUPS == 2 && CWAVES == 8) mfma_group(f1);
         }
@@ -724,7 +729,10 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
           store_loads(stg, true, gbuf ^ 1, wrap(base + XR), st + 1 < s_end);
           issue_loads(stg, c_next, true, 1);
         }
-        if (GROUPS == 2 && CWAVES != 8 && wave < CWAVES) mfma_group(f1);
+        if (GROUPS == 2 && CWAVES != 8 && wave < CWAVES) {
+          if (!kBothFirst) read_group(f1, gbuf, base, 1);
+          mfma_group(f1);
+        }
         if (st + 3 < s_end) advance(c_next);
         __syncthreads();
         if (st + 1 < s_end && c_store.hp == 0) {
