@@ -1,5 +1,6 @@
 // Host side of the small steps in native code: the distributed convolution (Step), ring attention over resident chunks, the
-// sharded LayerNorm's pieces between its collectives, GroupNorm of a whole tensor.
+// sharded LayerNorm's pieces between its collectives, GroupNorm of a whole tensor, the projections around attention and the
+// Swin block (SwinPass).
 //
 // The convolution: allocations, strips, pointer tables and the calls into
 // libjigsaw_hip.so, in native code. A step of one layer is 10 launches of 3 to 60 us; worked through Python
@@ -14,7 +15,12 @@
 // None before anything is launched; the callers' Python route then names the error or handles the case.
 #include <torch/extension.h>
 
+#include <algorithm>
 #include <atomic>
+#include <cmath>
+#include <memory>
+#include <tuple>
+#include <utility>
 #include <vector>
 
 #include "../../include/jigsaw_hip.h"
@@ -442,6 +448,250 @@ py::object gn_backward(const at::Tensor& g, const at::Tensor& x, const at::Tenso
   return py::make_tuple(given(gx), given(gw), given(gb));
 }
 
+// ---- projections around attention and the Swin block: the launches of projection.py and swin._WholeBlock in their order, for
+// tensors that need neither a cast nor a copy; None for all others, before anything is launched. Host time of a step, with
+// autograd's own: Swin block 573 us through Python, 334 here (its kernels take about 450 of 65536 tokens of 128 channels, less of
+// fewer); the two projections 213 and 164.
+struct Heads {  // (B, H, S, D) of the head layout
+  int64_t b = 1, h = 1, s = 1, d = 1;
+};
+
+at::Tensor f32(const at::Tensor& like, at::IntArrayRef shape) { return at::empty(shape, like.options().dtype(at::kFloat)); }
+at::Tensor bytes(const at::Tensor& like, size_t n) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
+
+// out(r, n) = sum_k a(r, k) w[n][k] (+ b[n])
+void nt(const at::Tensor& out, const at::Tensor& a, const at::Tensor& w, const at::Tensor* b, int64_t rows, bool a_heads, bool out_heads,
+        const Heads& l, void* s) {
+  check(jg_proj_nt(out.data_ptr(), a.data_ptr(), w.data_ptr(), b ? b->data_ptr() : nullptr, code_of(a), rows, w.size(0), w.size(1), a_heads, out_heads,
+                   l.b, l.h, l.s, l.d, s),
+        "jg_proj_nt");
+}
+void nt_fused(const at::Tensor& out, const at::Tensor& aux, int epilogue, const at::Tensor& a, const at::Tensor& w, const at::Tensor* b, int64_t rows, void* s) {
+  check(jg_proj_nt_fused(out.data_ptr(), aux.data_ptr(), epilogue, a.data_ptr(), w.data_ptr(), b ? b->data_ptr() : nullptr, code_of(a), rows, w.size(0),
+                         w.size(1), s),
+        "jg_proj_nt_fused");
+}
+// (gw, gb): gradients of a weight (n, c) and its bias from the gradient and the input of its layer
+std::pair<at::Tensor, at::Tensor> tn(const at::Tensor& g, const at::Tensor& x, int64_t rows, int64_t n, int64_t c, bool g_heads, bool x_heads, const Heads& l,
+                                     bool need_b, at::ScalarType grad_type, void* s) {
+  const auto options = g.options().dtype(grad_type);
+  const at::Tensor gw = at::empty({n, c}, options), gb = need_b ? at::empty({n}, options) : at::Tensor();
+  const size_t nbytes = jg_proj_tn_workspace(rows, n, c);
+  const at::Tensor ws = bytes(g, std::max<size_t>(nbytes, 16));
+  check(jg_proj_tn(gw.data_ptr(), need_b ? gb.data_ptr() : nullptr, g.data_ptr(), x.data_ptr(), code_of(g), grad_type == at::kFloat ? JG_F32 : code_of(g),
+                   rows, n, c, g_heads, x_heads, l.b, l.h, l.s, l.d, ws.data_ptr(), nbytes, s),
+        "jg_proj_tn");
+  return {gw, gb};
+}
+at::Tensor turned(const at::Tensor& w, void* s) {  // projection._transpose
+  const int64_t n = w.size(0), k = w.size(1);
+  if (w.element_size() != 2 || n % 8 != 0 || k % 8 != 0 || !aligned(w)) return w.t().contiguous();
+  const at::Tensor out = at::empty({k, n}, w.options());
+  check(jg_transpose16(out.data_ptr(), w.data_ptr(), n, k, s), "jg_transpose16");
+  return out;
+}
+
+bool projection_ok(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& b) {
+  return on_gpu(x) && on_gpu(w) && x.numel() > 0 && w.numel() > 0 && w.dim() == 2 && code_of(x) >= 0 && w.scalar_type() == x.scalar_type() &&
+         w.device() == x.device() &&
+         (!b || (on_gpu(*b) && b->dim() == 1 && b->size(0) == w.size(0) && b->scalar_type() == x.scalar_type() && b->device() == x.device()));
+}
+
+// (*lead, s, C) -> (3, *lead, heads, s, d)
+py::object qkv_forward(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& b, int64_t heads, uintptr_t stream) {
+  if (x.dim() < 2 || !projection_ok(x, w, b) || x.size(-1) != w.size(1) || heads < 1 || w.size(0) % (3 * heads) != 0) return py::none();
+  at::AutoDispatchBelowADInplaceOrView below;
+  const int64_t s = x.size(-2), rows = x.numel() / x.size(-1), d = w.size(0) / (3 * heads);
+  Shape shape{3};
+  shape.append(x.sizes().begin(), x.sizes().end() - 2);
+  for (int64_t v : {heads, s, d}) shape.push_back(v);
+  const at::Tensor out = at::empty(shape, x.options());
+  nt(out, x, w, b ? &*b : nullptr, rows, false, true, {rows / s, heads, s, d}, pointer(stream));
+  return py::cast(out);
+}
+
+// (*lead, heads, s, d) -> (*lead, s, n)
+py::object heads_forward(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& b, uintptr_t stream) {
+  if (x.dim() < 3 || !projection_ok(x, w, b) || x.size(-3) * x.size(-1) != w.size(1)) return py::none();
+  at::AutoDispatchBelowADInplaceOrView below;
+  const int64_t h = x.size(-3), s = x.size(-2), d = x.size(-1), rows = x.numel() / (h * d);
+  Shape shape(x.sizes().begin(), x.sizes().end() - 3);
+  for (int64_t v : {s, w.size(0)}) shape.push_back(v);
+  const at::Tensor out = at::empty(shape, x.options());
+  nt(out, x, w, b ? &*b : nullptr, rows, true, false, {rows / s, h, s, d}, pointer(stream));
+  return py::cast(out);
+}
+
+// (gx, gw, gb) of either; `qkv`: the gradient is in the head layout and x is not, else the other way round
+py::object projection_backward(const at::Tensor& g, const at::Tensor& x, const at::Tensor& w, bool qkv, int64_t b, int64_t h, int64_t sq, int64_t d,
+                               bool need_x, bool need_w, bool need_b, uintptr_t stream) {
+  const int64_t n = w.size(0), c = w.size(1), rows = b * sq;
+  if (!on_gpu(g) || !projection_ok(x, w, c10::nullopt) || g.scalar_type() != x.scalar_type() || g.device() != x.device() || g.numel() != rows * n ||
+      x.numel() != rows * c)
+    return py::none();
+  at::AutoDispatchBelowADInplaceOrView below;
+  void* const s = pointer(stream);
+  const Heads l{b, h, sq, d};
+  at::Tensor gx, gw, gb;
+  if (need_x) {
+    gx = at::empty_like(x);
+    nt(gx, g, turned(w, s), nullptr, rows, qkv, !qkv, l, s);
+  }
+  if (need_w || need_b) std::tie(gw, gb) = tn(g, x, rows, n, c, qkv, !qkv, l, need_b, g.scalar_type(), s);
+  auto given = [](const at::Tensor& t, bool wanted) -> py::object { return wanted ? py::cast(t) : py::none(); };
+  return py::make_tuple(given(gx, need_x), given(gw, need_w), given(gb, need_b));
+}
+
+// One pass of swin._WholeBlock with bf16 tokens and fp32 parameters on a grid that wraps inside the rank: what its backward reads.
+// The block's parameters in the order of swin._WholeBlock.forward.
+enum Param { N1W, N1B, QKV_W, QKV_B, TABLE, PROJ_W, PROJ_B, N2W, N2B, FC1_W, FC1_B, FC2_W, FC2_B, PARAMS };
+
+class SwinPass {
+ public:
+  // (result, pass) or None
+  static py::object forward(const at::Tensor& x, const List& p, const c10::optional<at::Tensor>& side, int64_t heads, int64_t shift, double eps,
+                            uintptr_t stream) {
+    if (x.dim() != 4 || x.numel() == 0 || !on_gpu(x) || !aligned(x) || x.scalar_type() != at::kBFloat16 || p.size() != PARAMS) return py::none();
+    const int64_t b = x.size(0), h = x.size(1), w = x.size(2), c = x.size(3), tokens = h * w, hidden = p[FC1_W].dim() == 2 ? p[FC1_W].size(0) : 0;
+    if (c != 32 * heads || h % 8 != 0 || w % 8 != 0 || hidden == 0 || hidden % 8 != 0 || !jg_ln_plain_supported(c)) return py::none();
+    const Shape want[PARAMS] = {{c}, {c}, {3 * c, c}, {3 * c}, {225, heads}, {c, c}, {c}, {c}, {c}, {hidden, c}, {hidden}, {c, hidden}, {c}};
+    for (int i = 0; i < PARAMS; ++i)
+      if (!on_gpu(p[i]) || p[i].scalar_type() != at::kFloat || p[i].device() != x.device() || p[i].sizes() != at::IntArrayRef(want[i])) return py::none();
+    if (side && (!on_gpu(*side) || side->scalar_type() != at::kByte || side->numel() != tokens || side->device() != x.device())) return py::none();
+    at::AutoDispatchBelowADInplaceOrView below;
+    auto pass = std::make_unique<SwinPass>();
+    SwinPass& t = *pass;
+    void* const s = pointer(stream);
+    const int64_t rows = b * tokens;
+    t.x = x, t.n1w = p[N1W], t.n2w = p[N2W], t.table = p[TABLE], t.l = {b, heads, tokens, 32}, t.h = h, t.w = w, t.shift = shift;
+    if (side) t.side = *side;
+    t.cast(p, s);
+    t.y1 = t.norm(x, p[N1W], p[N1B], t.mean1, t.rstd1, eps, s);
+    t.qkv = at::empty({3, b, heads, tokens, 32}, x.options());
+    nt(t.qkv, t.y1, t.wc[0], &t.bc[0], rows, false, true, t.l, s);
+    t.out = at::empty({b, heads, tokens, 32}, x.options());
+    t.lse = f32(x, {rows * heads});
+    const char* const q = static_cast<const char*>(t.qkv.data_ptr());
+    const int64_t part = 2 * rows * c;
+    check(jg_attn_swin_shifted_fwd(t.out.data_ptr(), t.lse.data_ptr<float>(), q, q + part, q + 2 * part, t.table.data_ptr<float>(), t.codes(), b, heads, h,
+                                   w, t.shift_y(), t.shift_x(), 32, (float)t.scale(), JG_BF16, s),
+          "jg_attn_swin_shifted_fwd");
+    t.x1 = at::empty_like(x);
+    check(jg_proj_nt_fused_heads(t.x1.data_ptr(), x.data_ptr(), JG_EPI_ADD, t.out.data_ptr(), t.wc[1].data_ptr(), t.bc[1].data_ptr(), JG_BF16, rows, c, c, 1, b,
+                                 heads, tokens, 32, s),
+          "jg_proj_nt_fused_heads");
+    t.y2 = t.norm(t.x1, p[N2W], p[N2B], t.mean2, t.rstd2, eps, s);
+    t.pre = at::empty({b, h, w, hidden}, x.options());
+    t.act = at::empty_like(t.pre);
+    nt_fused(t.pre, t.act, JG_EPI_GELU, t.y2, t.wc[2], &t.bc[2], rows, s);
+    const at::Tensor y = at::empty_like(x);
+    nt_fused(y, t.x1, JG_EPI_ADD, t.act, t.wc[3], &t.bc[3], rows, s);
+    return py::make_tuple(y, std::move(pass));
+  }
+
+  // Gradients of x (None unless wanted) and of the parameters, or None. The pass keeps nothing afterwards.
+  py::object backward(const at::Tensor& grad, bool need_x, uintptr_t stream) {
+    if (!x.defined() || grad.sizes() != x.sizes() || !on_gpu(grad) || !aligned(grad) || grad.scalar_type() != at::kBFloat16 || grad.device() != x.device())
+      return py::none();
+    at::AutoDispatchBelowADInplaceOrView below;
+    void* const s = pointer(stream);
+    const int64_t c = x.size(3), rows = l.b * l.s, hidden = pre.size(3);
+    const Heads flat;
+    at::Tensor g[PARAMS];
+    std::tie(g[FC2_W], g[FC2_B]) = tn(grad, act, rows, c, hidden, false, false, flat, true, at::kFloat, s);
+    const at::Tensor dpre = at::empty_like(pre);
+    nt_fused(dpre, pre, JG_EPI_DGELU, grad, wt[3], nullptr, rows, s);
+    std::tie(g[FC1_W], g[FC1_B]) = tn(dpre, y2, rows, hidden, c, false, false, flat, true, at::kFloat, s);
+    const at::Tensor gy2 = at::empty_like(x);
+    nt(gy2, dpre, wt[2], nullptr, rows, false, false, flat, s);
+    const at::Tensor gx1 = norm_backward(gy2, grad, x1, mean2, rstd2, n2w, true, &g[N2W], &g[N2B], s);
+    const at::Tensor gout = at::empty_like(out);
+    nt(gout, gx1, wt[1], nullptr, rows, false, true, l, s);
+    std::tie(g[PROJ_W], g[PROJ_B]) = tn(gx1, out, rows, c, c, false, true, l, true, at::kFloat, s);
+    const at::Tensor dqkv = at::empty_like(qkv);
+    g[TABLE] = at::empty_like(table);
+    const size_t nbytes = jg_attn_swin_bwd_workspace_bytes(l.b, l.h, h, w);
+    const at::Tensor ws = bytes(x, nbytes);
+    const char* const q = static_cast<const char*>(qkv.data_ptr());
+    char* const dq = static_cast<char*>(dqkv.data_ptr());
+    const int64_t part = 2 * rows * c;
+    check(jg_attn_swin_shifted_bwd(dq, dq + part, dq + 2 * part, g[TABLE].data_ptr<float>(), gout.data_ptr(), q, q + part, q + 2 * part, out.data_ptr(),
+                                   lse.data_ptr<float>(), table.data_ptr<float>(), codes(), l.b, l.h, h, w, shift_y(), shift_x(), 32, (float)scale(), JG_BF16,
+                                   ws.data_ptr(), nbytes, s),
+          "jg_attn_swin_shifted_bwd");
+    const at::Tensor gy = at::empty_like(x);
+    nt(gy, dqkv, wt[0], nullptr, rows, true, false, l, s);
+    std::tie(g[QKV_W], g[QKV_B]) = tn(dqkv, y1, rows, 3 * c, c, true, false, l, true, at::kFloat, s);
+    const at::Tensor gx = norm_backward(gy, gx1, x, mean1, rstd1, n1w, need_x, &g[N1W], &g[N1B], s);
+    py::tuple all(1 + PARAMS);
+    all[0] = need_x ? py::cast(gx) : py::none();
+    for (int i = 0; i < PARAMS; ++i) all[1 + i] = py::cast(g[i]);
+    *this = SwinPass();
+    return std::move(all);
+  }
+
+ private:
+  // bf16 copies of the four weights, their transposes and the biases in one launch (projection.cast_parameters)
+  void cast(const List& p, void* s) {
+    const int weight[4] = {QKV_W, PROJ_W, FC1_W, FC2_W}, bias[4] = {QKV_B, PROJ_B, FC1_B, FC2_B};
+    int64_t total = 0;
+    auto room = [&](const at::Tensor& t) { const int64_t at = total; total += (t.numel() + 7) / 8 * 8; return at; };
+    int64_t at_w[4], at_wt[4], at_b[4];
+    for (int i = 0; i < 4; ++i) at_w[i] = room(p[weight[i]]), at_wt[i] = room(p[weight[i]]), at_b[i] = room(p[bias[i]]);
+    const at::Tensor flat_ = at::empty({total}, x.options());
+    void *dst[8], *dst_t[8] = {};
+    const void* src[8];
+    int32_t rows[8], cols[8];
+    for (int i = 0; i < 4; ++i) {
+      const int64_t n = p[weight[i]].size(0), k = p[weight[i]].size(1);
+      wc[i] = at::as_strided(flat_, {n, k}, {k, 1}, at_w[i]);
+      wt[i] = at::as_strided(flat_, {k, n}, {n, 1}, at_wt[i]);
+      bc[i] = at::as_strided(flat_, {n}, {1}, at_b[i]);
+      dst[i] = wc[i].data_ptr(), dst_t[i] = wt[i].data_ptr(), src[i] = p[weight[i]].data_ptr(), rows[i] = n, cols[i] = k;
+      dst[4 + i] = bc[i].data_ptr(), src[4 + i] = p[bias[i]].data_ptr(), rows[4 + i] = 1, cols[4 + i] = n;
+    }
+    check(jg_cast_params(dst, dst_t, src, rows, cols, 8, s), "jg_cast_params");
+  }
+  static at::Tensor norm(const at::Tensor& x, const at::Tensor& w, const at::Tensor& b, at::Tensor& mean, at::Tensor& rstd, double eps, void* s) {
+    const int64_t cols = x.size(-1), rows = x.numel() / cols;
+    const at::Tensor y = at::empty_like(x);
+    mean = f32(x, {rows});
+    rstd = f32(x, {rows});
+    check(jg_ln_plain_fwd(y.data_ptr(), mean.data_ptr<float>(), rstd.data_ptr<float>(), x.data_ptr(), w.data_ptr<float>(), b.data_ptr<float>(), rows, cols,
+                          (float)eps, JG_BF16, JG_BF16, s),
+          "jg_ln_plain_fwd");
+    return y;
+  }
+  // the gradient of the norm's input with what reaches it past the norm (`over`) added, if wanted; gw, gb
+  static at::Tensor norm_backward(const at::Tensor& g, const at::Tensor& over, const at::Tensor& x, const at::Tensor& mean, const at::Tensor& rstd,
+                                  const at::Tensor& w, bool need_x, at::Tensor* gw, at::Tensor* gb, void* s) {
+    const int64_t cols = x.size(-1), rows = x.numel() / cols;
+    const at::Tensor gx = need_x ? at::empty_like(x) : at::Tensor();
+    *gw = f32(x, {cols});
+    *gb = f32(x, {cols});
+    const size_t nbytes = jg_ln_plain_bwd_workspace_bytes(rows, cols);
+    const at::Tensor ws = bytes(x, std::max<size_t>(nbytes, 4));
+    if (need_x)
+      check(jg_ln_plain_bwd_add(gx.data_ptr(), gw->data_ptr<float>(), gb->data_ptr<float>(), g.data_ptr(), x.data_ptr(), mean.data_ptr<float>(),
+                                rstd.data_ptr<float>(), w.data_ptr<float>(), rows, cols, JG_BF16, JG_BF16, ws.data_ptr(), nbytes, over.data_ptr(), s),
+            "jg_ln_plain_bwd_add");
+    else
+      check(jg_ln_plain_bwd(nullptr, gw->data_ptr<float>(), gb->data_ptr<float>(), g.data_ptr(), x.data_ptr(), mean.data_ptr<float>(),
+                            rstd.data_ptr<float>(), w.data_ptr<float>(), rows, cols, JG_BF16, JG_BF16, ws.data_ptr(), nbytes, s),
+            "jg_ln_plain_bwd");
+    return gx;
+  }
+  const uint8_t* codes() const { return side.defined() ? side.data_ptr<uint8_t>() : nullptr; }
+  int64_t shift_y() const { return (shift % h + h) % h; }
+  int64_t shift_x() const { return (shift % w + w) % w; }
+  static double scale() { return std::pow(32.0, -0.5); }
+
+  at::Tensor x, n1w, n2w, table, side, y1, mean1, rstd1, qkv, out, lse, x1, y2, mean2, rstd2, pre, act;
+  at::Tensor wc[4], wt[4], bc[4];  // qkv, output projection, the MLP's two layers
+  Heads l;
+  int64_t h = 0, w = 0, shift = 0;
+};
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -465,4 +715,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("ln_bwd_apply", &ln_bwd_apply);
   m.def("gn_forward", &gn_forward);
   m.def("gn_backward", &gn_backward);
+  m.def("qkv_forward", &qkv_forward);
+  m.def("heads_forward", &heads_forward);
+  m.def("projection_backward", &projection_backward);
+  py::class_<SwinPass>(m, "SwinPass").def("backward", &SwinPass::backward);
+  m.def("swin_forward", &SwinPass::forward);
 }

@@ -183,11 +183,34 @@ def _tn(g, x, rows, n, c, g_heads, x_heads, dims, want_bias, grad_dtype=None):
     return gw, gb
 
 
+def _native(*tensors):
+    """The native host module where it may take these tensors (parameters in the tokens' type, so that there is nothing to
+    cast or to remember), else ``None``."""
+    return _lib.host() if all(t is None or (t.is_cuda and t.dtype == tensors[0].dtype) for t in tensors) else None
+
+
+def _native_backward(ctx, grad, x, w, qkv: bool):
+    """``(gx, gw, gb)`` from the native host module for a pass whose forward it ran, or ``None``; a pass whose weights came
+    with their transposes (:func:`cast_parameters`) has fp32 parameters, which the native call does not know."""
+    if not getattr(ctx, "native", False) or _remember_casts or getattr(ctx, "weight_t", None) is not None:
+        return None
+    need = ctx.needs_input_grad
+    return _lib.host().projection_backward(grad, x, w, qkv, *ctx.dims, need[0], need[1], ctx.has_bias and need[2], _lib.stream_handle(x.device))
+
+
 class _QkvProjection(torch.autograd.Function):
     """``(*lead, s, C) -> (3, *lead, h, s, d)`` with ``weight (3 h d, C)``."""
 
     @staticmethod
     def forward(ctx, x, weight, bias, heads):  # noqa: D102
+        host = _native(x, weight, bias)
+        out = None if host is None else host.qkv_forward(x, weight, bias, heads, _lib.stream_handle(x.device))
+        if out is not None:
+            ctx.save_for_backward(x, weight)
+            ctx.weight_ref, ctx.weight_version = weight, weight._version
+            ctx.dims, ctx.has_bias = (x.numel() // (x.shape[-1] * x.shape[-2]), *out.shape[-3:]), bias is not None
+            ctx.dtypes, ctx.native = (weight.dtype, None if bias is None else bias.dtype), True
+            return out
         _lib.require_gpu(x, weight, bias)
         if x.dim() < 2:
             raise ValueError("x must be (..., seq, channels)")
@@ -215,6 +238,9 @@ class _QkvProjection(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad):  # noqa: D102
         xc, w = ctx.saved_tensors
+        got = _native_backward(ctx, grad, xc, w, True)
+        if got is not None:
+            return (*got, None)
         b, h, s, d = ctx.dims
         n_out, c = w.shape
         g = grad.to(xc.dtype).contiguous()
@@ -241,6 +267,15 @@ class _HeadsProjection(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, out, weight, bias, residual=None):  # noqa: D102
+        host = _native(out, weight, bias) if residual is None else None
+        y = None if host is None else host.heads_forward(out, weight, bias, _lib.stream_handle(out.device))
+        if y is not None:
+            ctx.save_for_backward(out, weight)
+            ctx.weight_ref, ctx.weight_version = weight, weight._version
+            h, s, d = out.shape[-3:]
+            ctx.dims, ctx.has_bias, ctx.has_residual = (out.numel() // (h * s * d), h, s, d), bias is not None, False
+            ctx.dtypes, ctx.native = (weight.dtype, None if bias is None else bias.dtype), True
+            return y
         _lib.require_gpu(out, weight, bias, residual)
         if out.dim() < 3:
             raise ValueError("out must be (..., heads, seq, head_dim)")
@@ -272,6 +307,9 @@ class _HeadsProjection(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad):  # noqa: D102
         oc, w = ctx.saved_tensors
+        got = _native_backward(ctx, grad, oc, w, False)
+        if got is not None:
+            return (*got, None)
         b, h, s, d = ctx.dims
         n_out, k = w.shape
         g = grad.to(oc.dtype).contiguous()

@@ -179,11 +179,21 @@ class _WholeBlock(torch.autograd.Function):
     def forward(ctx, x, n1w, n1b, qkv_w, qkv_b, table, proj_w, proj_b, n2w, n2b, w1, b1, w2, b2, block):  # noqa: D102
         b, h, w, c = x.shape
         dt, eps, heads = _compute_dtype(x), block.eps, block.attn.heads
+        wanted = tuple(ctx.needs_input_grad) if hasattr(ctx, "needs_input_grad") else (True,) * 15
+        roll = block.shift_by and not block.shift_is_local()
+        # in native code where the parameters are fp32 and all of them (or nothing) want a gradient: the same launches
+        host = _lib.host() if not roll and not casts_remembered() and n1b is not None and n2b is not None else None
+        if host is not None and (all(wanted[1:14]) or not any(wanted)):
+            got = host.swin_forward(x, (n1w, n1b, qkv_w, qkv_b, table, proj_w, proj_b, n2w, n2b, w1, b1, w2, b2), block.attn.side, heads,
+                                    block.shift_by, eps, _lib.stream_handle(x.device))
+            if got is not None:
+                ctx.stages, ctx.rolled, ctx.grid = got[1], False, (b, h, w, c)
+                return got[0]
         st = [_Stage() for _ in range(8)]
         # what each part has to differentiate: its parameters as autograd asks for them here (a frozen parameter
         # gets no gradient kernel where the part looks at the flag); the inputs between the parts always, x itself
         # only when it wants a gradient
-        nig = tuple(ctx.needs_input_grad) if hasattr(ctx, "needs_input_grad") else (True,) * 15
+        nig = wanted
         pad = (False,) * 6
         st[0].needs_input_grad = (nig[0], nig[1], nig[2]) + pad
         st[1].needs_input_grad = (True,) + pad
@@ -197,7 +207,6 @@ class _WholeBlock(torch.autograd.Function):
         one_cast = not casts_remembered() and all(t.dtype == torch.float32 and t.is_contiguous() for t in params)
         if one_cast:
             (qkv_w, proj_w, w1, w2), turned, (qkv_b, proj_b, b1, b2) = cast_parameters(params[::2], params[1::2])
-        roll = block.shift_by and not block.shift_is_local()
         y = _PlainLayerNormFork.forward(st[0], x, n1w, n1b, eps, dt)[0]
         if roll:
             y = _Roll.forward(st[1], y.contiguous(), (-block.shift_by,) * 2, (1, 2), *block._roll_args())
@@ -226,6 +235,11 @@ class _WholeBlock(torch.autograd.Function):
                 "retain_graph=True does not keep them). Run the forward again, or build the block with one_node=False."
             )
         st, (b, h, w, c) = ctx.stages, ctx.grid
+        if not isinstance(st, list):
+            ctx.stages = None
+            g = grad.to(torch.bfloat16).contiguous()
+            g = g if g.data_ptr() % 16 == 0 else g.clone()
+            return (*st.backward(g, ctx.needs_input_grad[0], _lib.stream_handle(grad.device)), None)
         gy2, gw1, gb1, gw2, gb2, over = _GeluMlp.backward(st[7], grad)
         gx1, gn2w, gn2b = _PlainLayerNormFork.backward(st[6], gy2, over)[:3]
         ga = _Roll.backward(st[5], gx1)[0] if ctx.rolled else gx1

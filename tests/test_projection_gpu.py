@@ -85,6 +85,34 @@ def test_projections_match_oracle(case, dev):
             assert rel_l2(bod.grad.cpu(), gb) <= tol
 
 
+@pytest.mark.parametrize("need", [(True, True, True), (True, False, False), (False, True, False), (False, False, True)])
+@pytest.mark.parametrize("case", CASES, ids=_id)
+def test_native_projections_have_the_bits_of_the_python_route(case, need, dev, monkeypatch):
+    lead, s, c, heads, d, n2, dtype, has_b = case
+    gen = torch.Generator(device=dev).manual_seed(22)
+    make = lambda *shape: torch.randn(*shape, device=dev, generator=gen).to(dtype)  # noqa: E731
+    x, w, b, g = make(*lead, s, c), make(3 * heads * d, c), make(3 * heads * d), make(3, *lead, heads, s, d)
+    o, wo, bo, g2 = make(*lead, heads, s, d), make(n2, heads * d), make(n2), make(*lead, s, n2)
+
+    def passes():
+        out = []
+        for call, args, grad in ((lambda *a: jp.qkv_projection(*a, heads), (x, w, b), g), (jp.heads_projection, (o, wo, bo), g2)):
+            leaves = [t.clone().requires_grad_(n) for t, n in zip(args, need)]
+            if not has_b:
+                leaves[2] = None
+            y = call(*leaves)
+            out.append(y.detach())
+            if y.requires_grad:
+                y.backward(grad)
+            out += [t.grad for t in leaves if t is not None]
+        return out
+
+    here = passes()
+    monkeypatch.setattr(jp._lib, "host", lambda: None)
+    for a, want in zip(here, passes()):
+        assert (a is None and want is None) or torch.equal(a, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_identity_weight_is_the_rearrange_exactly(dtype, dev):
     """With the identity as weight and no bias the projection only moves data: the

@@ -189,6 +189,33 @@ def test_block_as_one_autograd_node_has_the_bits_of_its_parts(shift, n, dev):
         assert rel_l2(prm.grad, params[name].grad) < 2e-2, name
 
 
+@pytest.mark.parametrize("batch,n,dim,shift", [(1, (8, 8), 64, 4), (2, (24, 40), 96, 0), (3, (32, 16), 256, 3)])
+def test_native_block_has_the_bits_of_the_python_route(batch, n, dim, shift, dev, monkeypatch):
+    """A gradient off the 16-byte grid and a pass without any gradient among them."""
+    torch.manual_seed(6)
+    block = js.SwinBlock(dim, dim // 32, 8, n, shift=shift, device=dev)
+    x = torch.randn(batch, *n, dim, device=dev).bfloat16()
+    g = torch.randn(x.numel() + 1, device=dev).bfloat16()[1:].view_as(x)
+
+    def passes():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            with torch.no_grad():
+                out = [block(x)]
+            xg = x.clone().requires_grad_()
+            y = block(xg)
+        return [*out, y, *torch.autograd.grad(y, (xg, *block.parameters()), g.clone())]
+
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        xg = x.clone().requires_grad_()
+        off = torch.autograd.grad(block(xg), (xg, *block.parameters()), g)
+    here = passes()
+    for a, want in zip(off, here[2:]):
+        assert torch.equal(a, want)
+    monkeypatch.setattr(js._lib, "host", lambda: None)
+    for a, want in zip(here, passes()):
+        assert torch.equal(a, want)
+
+
 @pytest.mark.parametrize("shift", [0, 4])
 def test_block_step_recorded_in_a_hip_graph_replays_the_eager_step(shift, dev):
     """``SwinBlock.captured_step``: forward + backward recorded once, replayed several times with eager
