@@ -39,10 +39,12 @@ struct SwinArgs {
   float* lse;                              // (entries, 64), entry = (image * windows + window) * heads + head
   const float* table;                      // (225, heads)
   const uint8_t* side;                     // (windows, 64) or NULL
-  float* bins;                             // (entries, 2, 225) or NULL: table-gradient parts
-  int heads, gh, gw, nwx, nwin;
+  float* bins;                             // (slots * heads, 2, 225) or NULL: table-gradient parts
+  int heads, gh, gw, nwx, nwin;            // nwin: windows of an image
   int shift_y, shift_x;                    // the windows lie on the grid rolled by minus this: 0 <= shift < gh, gw
-  long long entries, tokens;
+  unsigned entries;                        // < 2^31
+  long long tokens;
+  int slots;                               // backward: wavefronts per head
   float scale;
 };
 
@@ -52,14 +54,14 @@ struct Entry {
   int head, win;
 };
 
-__device__ inline Entry locate(const SwinArgs& p, long long e, int ln) {
+// e is the same in all lanes, and the callers see to it that the compiler knows (scalar divisions and bases).
+__device__ inline Entry locate(const SwinArgs& p, unsigned e, int ln) {
   Entry r;
-  r.head = (int)(e % p.heads);
-  const long long t = e / p.heads;
-  r.win = (int)(t % p.nwin);
-  const long long img = t / p.nwin;
+  const unsigned t = e / (unsigned)p.heads, img = t / (unsigned)p.nwin;
+  r.head = (int)(e - t * (unsigned)p.heads);
+  r.win = (int)(t - img * (unsigned)p.nwin);
   const int wy = r.win / p.nwx, wx = r.win - wy * p.nwx;
-  r.base = (img * p.heads + r.head) * p.tokens * D;
+  r.base = ((long long)img * p.heads + r.head) * p.tokens * D;
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
     int y = wy * WIN + 4 * b + (ln >> 3) + p.shift_y, x = wx * WIN + (ln & 7) + p.shift_x;
@@ -105,9 +107,9 @@ __device__ inline uint64_t apart_from(const Sides& s, int mine) {
 // ------------------------------------------------------------------- forward
 __global__ __launch_bounds__(WAVES * 64) void attn_swin_fwd_kernel(SwinArgs p) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[WAVES * (TILE + 1024)];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 31, kg = lane >> 5;
-  long long e = (long long)blockIdx.x * WAVES + wave;
+  unsigned e = blockIdx.x * WAVES + wave;
   const bool valid = e < p.entries;
   if (!valid) e = p.entries - 1;  // computed again, not stored: every wavefront reaches the barrier
   const Entry en = locate(p, e, ln);
@@ -182,7 +184,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_swin_fwd_kernel(SwinArgs p) {
       uint16_t* orow = p.o + en.base + en.rowoff[nb];
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4) *reinterpret_cast<u32x2*>(orow + i4 * 8 + kg * 4) = pack_rows(o, i4, inv);
-      if (kg == 0) p.lse[e * N + qi] = sum > 0.0f ? ms * LN2 + __logf(sum) : -INFINITY;
+      if (kg == 0) p.lse[(size_t)e * N + qi] = sum > 0.0f ? ms * LN2 + __logf(sum) : -INFINITY;
     }
   }
 }
@@ -192,15 +194,49 @@ constexpr int BINS = 2 * ROWS;  // per wavefront: one set per lane half
 constexpr int BWD_PER_WAVE = 3 * TILE + 2 * N * 4 + 1024 + (BINS * 4 + 15) / 16 * 16;  // 18704
 constexpr int BWD_LDS = WAVES * BWD_PER_WAVE;                                            // 74816
 
+// A wavefront takes every slots-th window of one head: the table and the bins stay in its LDS, and the rows of
+// its next window are on their way while it works on this one (a window is 1.5 us of dependent LDS accesses
+// and matrix instructions behind 24 KB of loads, with two wavefronts a SIMD). All LDS is the wavefront's own.
+struct WindowRows {
+  Entry en;
+  bf16x8 k[2][2], q[2][2], v[2][2], dout[2][2], out[2][2];
+  float lse[2];
+};
+__device__ inline void load_window(WindowRows& w, const SwinArgs& p, unsigned e, int ln, int kg) {
+  w.en = locate(p, e, ln);
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      w.k[b][ks] = load_row(p.k + w.en.base, w.en.rowoff[b], ks, kg);
+      w.q[b][ks] = load_row(p.q + w.en.base, w.en.rowoff[b], ks, kg);
+      w.v[b][ks] = load_row(p.v + w.en.base, w.en.rowoff[b], ks, kg);
+      w.dout[b][ks] = load_row(p.dout + w.en.base, w.en.rowoff[b], ks, kg);
+      w.out[b][ks] = load_row(p.out + w.en.base, w.en.rowoff[b], ks, kg);
+    }
+    w.lse[b] = p.lse[(size_t)e * N + b * 32 + ln];
+  }
+}
+// Block b of a tile in LDS as fragments again: in registers beside the next window's rows they would spill.
+__device__ inline void tile_rows(bf16x8 (&f)[2], const unsigned char* tile, int b, int ln, int kg) {
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+    f[ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(tile + (b * 32 + ln) * PITCH + (ks * 16 + kg * 8) * 2));
+}
+// Between LDS accesses of different lanes of one wavefront: the LDS keeps their order, the compiler has to.
+__device__ inline void lanes_in_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 template <bool DTABLE>
-__global__ __launch_bounds__(WAVES * 64) void attn_swin_bwd_kernel(SwinArgs p) {
+__global__ __launch_bounds__(WAVES * 64, 2) void attn_swin_bwd_kernel(SwinArgs p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 31, kg = lane >> 5;
-  long long e = (long long)blockIdx.x * WAVES + wave;
-  const bool valid = e < p.entries;
-  if (!valid) e = p.entries - 1;
-  const Entry en = locate(p, e, ln);
+  const unsigned worker = blockIdx.x * WAVES + wave;
+  const unsigned step = (unsigned)p.slots * (unsigned)p.heads;
+  if (worker >= step) return;
   unsigned char* kt = smem + wave * BWD_PER_WAVE;
   unsigned char* qt = kt + TILE;
   unsigned char* dot = qt + TILE;
@@ -209,154 +245,158 @@ __global__ __launch_bounds__(WAVES * 64) void attn_swin_bwd_kernel(SwinArgs p) {
   float* tab = delta_s + N;
   float* bins = tab + 256;
 
-  bf16x8 kf[2][2], qf[2][2], vf[2][2], dof[2][2];
-#pragma unroll
-  for (int b = 0; b < 2; ++b)
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      kf[b][ks] = load_row(p.k + en.base, en.rowoff[b], ks, kg);
-      qf[b][ks] = load_row(p.q + en.base, en.rowoff[b], ks, kg);
-      vf[b][ks] = load_row(p.v + en.base, en.rowoff[b], ks, kg);
-      dof[b][ks] = load_row(p.dout + en.base, en.rowoff[b], ks, kg);
-    }
-  load_table(tab, p, en.head, lane);
-  const Sides sd = load_sides(p, en.win, lane);
+  WindowRows next;
+  load_window(next, p, worker, ln, kg);
+  load_table(tab, p, next.en.head, lane);
   if (DTABLE)
     for (int i = lane; i < BINS; i += 64) bins[i] = 0.0f;
-  store_tile(kt, kf, ln, kg);
-  store_tile(qt, qf, ln, kg);
-  store_tile(dot, dof, ln, kg);
 
-  // delta = rowsum(dout * out) and lse (in base 2) of this lane's queries
-  float delta_q[2], lse_q[2];
+  for (unsigned e = worker; e < p.entries; e += step) {
+    const Entry en = next.en;
+    bf16x8 vf[2][2];
 #pragma unroll
-  for (int nb = 0; nb < 2; ++nb) {
-    const int qi = nb * 32 + ln;
-    float part = 0.0f;
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const bf16x8 of = load_row(p.out + en.base, en.rowoff[nb], ks, kg);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) part += (float)dof[nb][ks][j] * (float)of[j];
-    }
-    part += __shfl_xor(part, 32, 64);
-    delta_q[nb] = part;
-    lse_q[nb] = p.lse[e * N + qi] * LOG2E;
-    if (kg == 0) {
-      delta_s[qi] = part;
-      lse_s[qi] = lse_q[nb];
-    }
-  }
-  __syncthreads();
+      for (int ks = 0; ks < 2; ++ks) vf[b][ks] = next.v[b][ks];
+    const Sides sd = load_sides(p, en.win, lane);
+    lanes_in_order();
+    store_tile(kt, next.k, ln, kg);
+    store_tile(qt, next.q, ln, kg);
+    store_tile(dot, next.dout, ln, kg);
 
-  const float c2 = p.scale * LOG2E;
-
-  // ---- pass A: lane = query
+    // delta = rowsum(dout * out) and lse (in base 2) of this lane's queries
+    float delta_q[2], lse_q[2];
 #pragma unroll
-  for (int nb = 0; nb < 2; ++nb) {
-    const int qi = nb * 32 + ln;
-    f32x16 s[2] = {zero16(), zero16()}, dp[2] = {zero16(), zero16()};
+    for (int nb = 0; nb < 2; ++nb) {
+      const int qi = nb * 32 + ln;
+      float part = 0.0f;
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+      for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        s[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[mb][ks], qf[nb][ks], s[mb], 0, 0, 0);
-        dp[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[mb][ks], dof[nb][ks], dp[mb], 0, 0, 0);
+        for (int j = 0; j < 8; ++j) part += (float)next.dout[nb][ks][j] * (float)next.out[nb][ks][j];
+      part += __shfl_xor(part, 32, 64);
+      delta_q[nb] = part;
+      lse_q[nb] = next.lse[nb] * LOG2E;
+      if (kg == 0) {
+        delta_s[qi] = part;
+        lse_s[qi] = lse_q[nb];
       }
-    const int row0 = 15 * (qi >> 3) + (qi & 7) + 112 - 4 * kg - TOP;
-    const float* tl = tab + row0;
-    float* bl = bins + kg * ROWS + row0;
-    const uint64_t ap = sd.mixed ? apart_from(sd, qi) >> (4 * kg) : 0ull;
-    f32x16 dqa = zero16();
-    float ds[2][16];
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb) {
-      const uint32_t word = (uint32_t)(ap >> (32 * mb));
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int i = i4 * 4 + r;
-          const int c = TOP - (60 * mb + 15 * i4 + r);
-          float pr = __builtin_amdgcn_exp2f(s[mb][i] * c2 + tl[c] - lse_q[nb]);
-          if (sd.mixed && ((word >> (8 * i4 + r)) & 1u)) pr = 0.0f;
-          ds[mb][i] = pr * (dp[mb][i] - delta_q[nb]);
-        }
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        dqa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(kt, mb * 2 + h, ln, kg), pack_half(ds[mb], h), dqa, 0, 0, 0);
     }
-    if (DTABLE && valid) {
-      // dS^T into the bins, register by register: the 32 lanes of a half hit 32 different rows, and
-      // so do a register of key block 0 and its twin of block 1 (their rows differ by 60, more
-      // than the queries of a 32-lane block are apart), so the pair is read, added to and
-      // written back as plain LDS accesses; the LDS keeps a wavefront's accesses in order.
-      // (LDS float atomics do the same job at about 800 cycles an instruction.)
+    lanes_in_order();
+
+    const float c2 = p.scale * LOG2E;
+
+    // ---- pass A: lane = query
+    bf16x8 kf[2][2];
+    tile_rows(kf[0], kt, 0, ln, kg);
+    tile_rows(kf[1], kt, 1, ln, kg);
 #pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4)
+    for (int nb = 0; nb < 2; ++nb) {
+      const int qi = nb * 32 + ln;
+      __builtin_amdgcn_sched_barrier(0);
+      bf16x8 qf[2], dof[2];
+      tile_rows(qf, qt, nb, ln, kg);
+      tile_rows(dof, dot, nb, ln, kg);
+      const int row0 = 15 * (qi >> 3) + (qi & 7) + 112 - 4 * kg - TOP;
+      const float* tl = tab + row0;
+      float* bl = bins + kg * ROWS + row0;
+      const uint64_t ap = sd.mixed ? apart_from(sd, qi) >> (4 * kg) : 0ull;
+      f32x16 dqa = zero16();
+      float ds[2][16];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int i = i4 * 4 + r;
-          const int c0 = TOP - (15 * i4 + r), c1 = c0 - 60;
-          const float b0 = bl[c0], b1 = bl[c1];
-          bl[c0] = b0 + ds[0][i];
-          bl[c1] = b1 + ds[1][i];
-          // for one lane the rows of different registers never coincide, so the compiler would be
-          // free to read ahead; other lanes' rows do coincide with them: one step after the other
-          asm volatile("" ::: "memory");
+      for (int mb = 0; mb < 2; ++mb) {
+        f32x16 s = zero16(), dp = zero16();
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[mb][ks], qf[ks], s, 0, 0, 0);
+          dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[mb][ks], dof[ks], dp, 0, 0, 0);
         }
-    }
-    if (valid) {
+        const uint32_t word = (uint32_t)(ap >> (32 * mb));
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int i = i4 * 4 + r;
+            const int c = TOP - (60 * mb + 15 * i4 + r);
+            float pr = __builtin_amdgcn_exp2f(s[i] * c2 + tl[c] - lse_q[nb]);
+            if (sd.mixed && ((word >> (8 * i4 + r)) & 1u)) pr = 0.0f;
+            ds[mb][i] = pr * (dp[i] - delta_q[nb]);
+          }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          dqa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(kt, mb * 2 + h, ln, kg), pack_half(ds[mb], h), dqa, 0, 0, 0);
+      }
+      if (DTABLE) {
+        // dS^T into the bins, register by register: the 32 lanes of a half hit 32 different rows, and
+        // so do a register of key block 0 and its twin of block 1 (their rows differ by 60, more
+        // than the queries of a 32-lane block are apart), so the pair is read, added to and
+        // written back as plain LDS accesses; the LDS keeps a wavefront's accesses in order.
+        // (LDS float atomics do the same job at about 800 cycles an instruction.)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int i = i4 * 4 + r;
+            const int c0 = TOP - (15 * i4 + r), c1 = c0 - 60;
+            const float b0 = bl[c0], b1 = bl[c1];
+            bl[c0] = b0 + ds[0][i];
+            bl[c1] = b1 + ds[1][i];
+            // for one lane the rows of different registers never coincide, so the compiler would be
+            // free to read ahead; other lanes' rows do coincide with them: one step after the other
+            asm volatile("" ::: "memory");
+          }
+      }
       uint16_t* row = p.dq + en.base + en.rowoff[nb];
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4) *reinterpret_cast<u32x2*>(row + i4 * 8 + kg * 4) = pack_rows(dqa, i4, p.scale);
     }
-  }
-  if (DTABLE && valid) {
-    float* dst = p.bins + e * BINS;
-    for (int i = lane; i < BINS; i += 64) dst[i] = bins[i];
-  }
 
-  // ---- pass B: lane = key
+    // in flight during pass B; pass A has no registers for them beside the table's gradient
+    if (e + step < p.entries) load_window(next, p, e + step, ln, kg);
+
+    // ---- pass B: lane = key
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int nbk = 0; nbk < 2; ++nbk) {
-    const int ki = nbk * 32 + ln;
-    f32x16 s[2] = {zero16(), zero16()}, dp[2] = {zero16(), zero16()};
+    for (int nbk = 0; nbk < 2; ++nbk) {
+      const int ki = nbk * 32 + ln;
+      __builtin_amdgcn_sched_barrier(0);
+      // table row of (query 32 mbq + 8 i4 + 4 kg + r, key ki) = 112 + 4 kg - 15 ky - kx + (60 mbq + 15 i4 + r)
+      const float* tl = tab + (112 + 4 * kg - 15 * (ki >> 3) - (ki & 7));
+      const uint64_t ap = sd.mixed ? apart_from(sd, ki) >> (4 * kg) : 0ull;
+      f32x16 dva = zero16(), dka = zero16();
 #pragma unroll
-    for (int mbq = 0; mbq < 2; ++mbq)
+      for (int mbq = 0; mbq < 2; ++mbq) {
+        const uint32_t word = (uint32_t)(ap >> (32 * mbq));
+        __builtin_amdgcn_sched_barrier(0);
+        bf16x8 qf[2], dof[2];
+        tile_rows(qf, qt, mbq, ln, kg);
+        tile_rows(dof, dot, mbq, ln, kg);
+        f32x16 s = zero16(), dp = zero16();
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        s[mbq] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[mbq][ks], kf[nbk][ks], s[mbq], 0, 0, 0);
-        dp[mbq] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dof[mbq][ks], vf[nbk][ks], dp[mbq], 0, 0, 0);
-      }
-    // table row of (query 32 mbq + 8 i4 + 4 kg + r, key ki) = 112 + 4 kg - 15 ky - kx + (60 mbq + 15 i4 + r)
-    const float* tl = tab + (112 + 4 * kg - 15 * (ki >> 3) - (ki & 7));
-    const uint64_t ap = sd.mixed ? apart_from(sd, ki) >> (4 * kg) : 0ull;
-    f32x16 dva = zero16(), dka = zero16();
+        for (int ks = 0; ks < 2; ++ks) {
+          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[ks], kf[nbk][ks], s, 0, 0, 0);
+          dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dof[ks], vf[nbk][ks], dp, 0, 0, 0);
+        }
+        float pr[16], ds[16];
 #pragma unroll
-    for (int mbq = 0; mbq < 2; ++mbq) {
-      const uint32_t word = (uint32_t)(ap >> (32 * mbq));
-      float pr[16], ds[16];
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const int q0 = mbq * 32 + i4 * 8 + kg * 4;
+          const f32x4 l4 = *reinterpret_cast<const f32x4*>(lse_s + q0);
+          const f32x4 d4 = *reinterpret_cast<const f32x4*>(delta_s + q0);
 #pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const int q0 = mbq * 32 + i4 * 8 + kg * 4;
-        const f32x4 l4 = *reinterpret_cast<const f32x4*>(lse_s + q0);
-        const f32x4 d4 = *reinterpret_cast<const f32x4*>(delta_s + q0);
+          for (int r = 0; r < 4; ++r) {
+            const int i = i4 * 4 + r;
+            pr[i] = __builtin_amdgcn_exp2f(s[i] * c2 + tl[60 * mbq + 15 * i4 + r] - l4[r]);
+            if (sd.mixed && ((word >> (8 * i4 + r)) & 1u)) pr[i] = 0.0f;
+            ds[i] = pr[i] * (dp[i] - d4[r]);
+          }
+        }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int i = i4 * 4 + r;
-          pr[i] = __builtin_amdgcn_exp2f(s[mbq][i] * c2 + tl[60 * mbq + 15 * i4 + r] - l4[r]);
-          if (sd.mixed && ((word >> (8 * i4 + r)) & 1u)) pr[i] = 0.0f;
-          ds[i] = pr[i] * (dp[mbq][i] - d4[r]);
+        for (int h = 0; h < 2; ++h) {
+          dva = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(dot, mbq * 2 + h, ln, kg), pack_half(pr, h), dva, 0, 0, 0);
+          dka = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(qt, mbq * 2 + h, ln, kg), pack_half(ds, h), dka, 0, 0, 0);
         }
       }
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        dva = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(dot, mbq * 2 + h, ln, kg), pack_half(pr, h), dva, 0, 0, 0);
-        dka = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(qt, mbq * 2 + h, ln, kg), pack_half(ds, h), dka, 0, 0, 0);
-      }
-    }
-    if (valid) {
       uint16_t* vrow = p.dv + en.base + en.rowoff[nbk];
       uint16_t* krow = p.dk + en.base + en.rowoff[nbk];
 #pragma unroll
@@ -366,20 +406,26 @@ __global__ __launch_bounds__(WAVES * 64) void attn_swin_bwd_kernel(SwinArgs p) {
       }
     }
   }
+  if (DTABLE) {
+    lanes_in_order();
+    float* dst = p.bins + (size_t)worker * BINS;
+    for (int i = lane; i < BINS; i += 64) dst[i] = bins[i];
+  }
 }
 
-// Table gradient, stage 1: block (head, chunk) adds the bins of its entries, entry after entry;
+// Table gradient, stage 1: block (head, chunk) adds the bins of its wavefronts, one after the other;
 // thread i < 450 owns bin i. stage 2: block `head` adds the chunks and the two lane halves.
 constexpr int CHUNKS = 32;
 __global__ __launch_bounds__(512) void swin_bins_stage1(const float* __restrict__ bins, float* __restrict__ part,
-                                                        long long entries, int heads) {
+                                                        long long workers, int heads) {
   const int head = blockIdx.x, chunk = blockIdx.y, i = threadIdx.x;
   if (i >= BINS) return;
-  const long long groups = entries / heads;  // entries of one head
+  const long long groups = workers / heads;  // wavefronts of one head
   const long long per = (groups + CHUNKS - 1) / CHUNKS;
   long long g0 = chunk * per, g1 = g0 + per;
   if (g1 > groups) g1 = groups;
   float acc = 0.0f;
+#pragma unroll 8
   for (long long g = g0; g < g1; ++g) acc += bins[(g * heads + head) * BINS + i];
   part[((size_t)head * CHUNKS + chunk) * BINS + i] = acc;
 }
@@ -404,6 +450,8 @@ int check(const char* who, int64_t images, int64_t heads, int64_t gh, int64_t gw
              "%s: the token grid (%lld x %lld) must be whole windows of %d x %d", who, (long long)gh, (long long)gw, WIN, WIN);
   JG_REQUIRE(gh * gw * D < (1ll << 31), "%s: token grid too large for 32-bit row offsets", who);
   JG_REQUIRE(scale > 0.0f, "%s: scale must be positive", who);
+  // (a tensor of 2^31 entries has 8 TB)
+  JG_REQUIRE(images < (1ll << 31) && images * heads < (1ll << 31) && images * heads * (gh / WIN) * (gw / WIN) < (1ll << 31), "%s: too many windows", who);
   return JG_OK;
 }
 
@@ -425,7 +473,7 @@ SwinArgs common(int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t s
   a.gw = (int)gw;
   a.nwx = (int)(gw / WIN);
   a.nwin = (int)((gh / WIN) * (gw / WIN));
-  a.entries = images * a.nwin * heads;
+  a.entries = (unsigned)(images * a.nwin * heads);
   a.tokens = gh * gw;
   a.scale = scale;
   return a;
@@ -451,7 +499,6 @@ extern "C" int jg_attn_swin_shifted_fwd(void* out, float* lse, const void* q, co
   a.v = static_cast<const uint16_t*>(v);
   a.o = static_cast<uint16_t*>(out);
   a.lse = lse;
-  JG_REQUIRE((a.entries + WAVES - 1) / WAVES < (1ll << 31), "%s: too many windows", who);
   attn_swin_fwd_kernel<<<dim3((unsigned)((a.entries + WAVES - 1) / WAVES)), WAVES * 64, 0, static_cast<hipStream_t>(stream)>>>(a);
   JG_CHECK_LAUNCH(who);
   return JG_OK;
@@ -490,9 +537,13 @@ extern "C" int jg_attn_swin_shifted_bwd(void* dq, void* dk, void* dv, float* dta
   a.dv = static_cast<uint16_t*>(dv);
   a.lse = const_cast<float*>(lse);
   a.bins = static_cast<float*>(workspace);
-  JG_REQUIRE((a.entries + WAVES - 1) / WAVES < (1ll << 31), "%s: too many windows", who);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)((a.entries + WAVES - 1) / WAVES));
+  // As many wavefronts as the device holds at a time (256 compute units, two workgroups each by LDS),
+  // the same number for every head.
+  const long long windows = a.entries / heads, most = (512ll * WAVES) / heads;
+  a.slots = (int)(most < 1 ? 1 : windows < most ? windows : most);
+  const long long workers = (long long)a.slots * heads;
+  const dim3 grid((unsigned)((workers + WAVES - 1) / WAVES));
   static bool lds_set = false;
   if (!lds_set) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_swin_bwd_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, BWD_LDS) != hipSuccess ||
@@ -503,8 +554,8 @@ extern "C" int jg_attn_swin_shifted_bwd(void* dq, void* dk, void* dv, float* dta
   if (dtable != nullptr) {
     attn_swin_bwd_kernel<true><<<grid, WAVES * 64, BWD_LDS, s>>>(a);
     JG_CHECK_LAUNCH(who);
-    float* part = a.bins + (size_t)a.entries * BINS;
-    swin_bins_stage1<<<dim3((unsigned)heads, CHUNKS), 512, 0, s>>>(a.bins, part, a.entries, (int)heads);
+    float* part = a.bins + (size_t)workers * BINS;
+    swin_bins_stage1<<<dim3((unsigned)heads, CHUNKS), 512, 0, s>>>(a.bins, part, workers, (int)heads);
     JG_CHECK_LAUNCH(who);
     swin_bins_stage2<<<dim3((unsigned)heads), 256, 0, s>>>(part, dtable, (int)heads);
     JG_CHECK_LAUNCH(who);

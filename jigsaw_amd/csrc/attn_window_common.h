@@ -36,15 +36,21 @@ __device__ inline void store_tile(unsigned char* tile, const bf16x8 (&f)[2][2], 
       *reinterpret_cast<u32x4*>(tile + (b * 32 + ln) * PITCH + (ks * 16 + kg * 8) * 2) = __builtin_bit_cast(u32x4, f[b][ks]);
 }
 
-// Transposed A fragment of K-step t: slot j = element [16 t + 8 (j / 4) + 4 kg + j % 4][ln].
+// Transposed A fragment of K-step t: slot j = element [16 t + 8 (j / 4) + 4 kg + j % 4][ln], by two LDS
+// transpose reads (within 16 lanes, lane i receives element i % 4 of the 8 bytes that lanes i / 4 + 4 j
+// point at, j = 0..3) in place of eight 2-byte reads, which were most of these kernels' LDS instructions.
 __device__ inline bf16x8 frag_tr(const unsigned char* tile, int t, int ln, int kg) {
-  bf16x8 r;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int row = t * 16 + (j >> 2) * 8 + kg * 4 + (j & 3);
-    r[j] = *reinterpret_cast<const __bf16*>(tile + row * PITCH + ln * 2);
-  }
-  return r;
+  typedef short i16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) i16x4* tr_ptr;
+  const unsigned char* const at = tile + (4 * kg + ((ln >> 2) & 3)) * PITCH + (ln >> 4) * 32 + (ln & 3) * 8 + t * (16 * PITCH);
+  const i16x4 l = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at));
+  const i16x4 h = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at + 8 * PITCH));
+  u32x4 w;
+  w.x = __builtin_bit_cast(u32x2, l).x;
+  w.y = __builtin_bit_cast(u32x2, l).y;
+  w.z = __builtin_bit_cast(u32x2, h).x;
+  w.w = __builtin_bit_cast(u32x2, h).y;
+  return __builtin_bit_cast(bf16x8, w);
 }
 
 // Slots of K-step h (0 / 1) of a 32-row accumulator block, rounded to bf16.

@@ -107,6 +107,28 @@ def test_windows_of_a_rolled_grid_without_the_roll(grid, shift, dev):
     assert torch.equal(out, rolled(want, shift)) and torch.equal(da, rolled(dr, shift)) and torch.equal(dta, dtr)
 
 
+@pytest.mark.parametrize("batch,heads,grid,shift", [(2, 5, (136, 128), 4), (3, 3, (256, 128), 0), (1, 2100, (8, 16), 0)])
+def test_more_windows_than_wavefronts(batch, heads, grid, shift, dev):
+    """Backward wavefronts that take several windows each, some one more than others: the gradients have the bits of
+    smaller calls whose wavefronts take one, and the table's gradient is their sum up to the order of fp32 sums
+    (2^-24 times the square root of 544 additions, some of them cancelling: 1e-5)."""
+    torch.manual_seed(7)
+    gh, gw = grid
+    qkv = torch.randn(3, batch, heads, gh * gw, 32, device=dev).bfloat16().requires_grad_()
+    table = (torch.randn(225, heads, device=dev) * 0.5).requires_grad_()
+    side = js.border_sides(gh, gw, 8, shift, (TileGroup(1, 0), TileGroup(1, 0))).to(torch.uint8).to(dev) if shift else None
+    g = torch.randn(batch, heads, gh * gw, 32, device=dev).bfloat16()
+    dqkv, dtable = torch.autograd.grad(ja.swin_grid_attention_packed(qkv, table, side, grid, shift), (qkv, table), g)
+    total = torch.zeros(225, heads, dtype=torch.float64, device=dev)
+    for i in range(batch):
+        for h in range(0, heads, 700):
+            part, t = qkv.detach()[:, i : i + 1, h : h + 700].contiguous().requires_grad_(), table.detach()[:, h : h + 700].contiguous().requires_grad_()
+            d, dt = torch.autograd.grad(ja.swin_grid_attention_packed(part, t, side, grid, shift), (part, t), g[i : i + 1, h : h + 700].contiguous())
+            assert torch.equal(d, dqkv[:, i : i + 1, h : h + 700])
+            total[:, h : h + 700] += dt
+    assert rel_l2(dtable, total) < 1e-5
+
+
 def test_parameters_cast_in_one_launch(dev):
     """bf16 copies and transposes of fp32 matrices whose edges are no multiples of the 64-wide tiles."""
     from jigsaw_amd.projection import cast_parameters
