@@ -278,7 +278,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_swin_bwd_kernel(SwinArgs p
       delta_q[nb] = part;
       lse_q[nb] = next.lse[nb] * LOG2E;
       if (kg == 0) {
-        delta_s[qi] = part;
+        delta_s[qi] = -part;
         lse_s[qi] = lse_q[nb];
       }
     }
@@ -305,23 +305,27 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_swin_bwd_kernel(SwinArgs p
       float ds[2][16];
 #pragma unroll
       for (int mb = 0; mb < 2; ++mb) {
-        f32x16 s = zero16(), dp = zero16();
+        f32x16 s = zero16(), dp;  // dp: less delta from the start
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dp[i] = -delta_q[nb];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
           s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[mb][ks], qf[ks], s, 0, 0, 0);
           dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[mb][ks], dof[ks], dp, 0, 0, 0);
         }
-        const uint32_t word = (uint32_t)(ap >> (32 * mb));
+        float x[16];
 #pragma unroll
         for (int i4 = 0; i4 < 4; ++i4)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int i = i4 * 4 + r;
-            const int c = TOP - (60 * mb + 15 * i4 + r);
-            float pr = __builtin_amdgcn_exp2f(s[i] * c2 + tl[c] - lse_q[nb]);
-            if (sd.mixed && ((word >> (8 * i4 + r)) & 1u)) pr = 0.0f;
-            ds[mb][i] = pr * (dp[i] - delta_q[nb]);
-          }
+          for (int r = 0; r < 4; ++r) x[i4 * 4 + r] = s[i4 * 4 + r] * c2 + tl[TOP - (60 * mb + 15 * i4 + r)] - lse_q[nb];
+        if (sd.mixed) {  // wave-uniform
+          const uint32_t word = (uint32_t)(ap >> (32 * mb));
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if ((word >> (8 * (i >> 2) + (i & 3))) & 1u) x[i] = -INFINITY;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) ds[mb][i] = __builtin_amdgcn_exp2f(x[i]) * dp[i];
 #pragma unroll
         for (int h = 0; h < 2; ++h)
           dqa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_tr(kt, mb * 2 + h, ln, kg), pack_half(ds[mb], h), dqa, 0, 0, 0);
@@ -366,30 +370,39 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_swin_bwd_kernel(SwinArgs p
       f32x16 dva = zero16(), dka = zero16();
 #pragma unroll
       for (int mbq = 0; mbq < 2; ++mbq) {
-        const uint32_t word = (uint32_t)(ap >> (32 * mbq));
         __builtin_amdgcn_sched_barrier(0);
         bf16x8 qf[2], dof[2];
         tile_rows(qf, qt, mbq, ln, kg);
         tile_rows(dof, dot, mbq, ln, kg);
-        f32x16 s = zero16(), dp = zero16();
+        f32x16 s = zero16(), dp;
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const f32x4 d4 = *reinterpret_cast<const f32x4*>(delta_s + mbq * 32 + i4 * 8 + kg * 4);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) dp[i4 * 4 + r] = d4[r];
+        }
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
           s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[ks], kf[nbk][ks], s, 0, 0, 0);
           dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dof[ks], vf[nbk][ks], dp, 0, 0, 0);
         }
-        float pr[16], ds[16];
+        float x[16], pr[16], ds[16];
 #pragma unroll
         for (int i4 = 0; i4 < 4; ++i4) {
-          const int q0 = mbq * 32 + i4 * 8 + kg * 4;
-          const f32x4 l4 = *reinterpret_cast<const f32x4*>(lse_s + q0);
-          const f32x4 d4 = *reinterpret_cast<const f32x4*>(delta_s + q0);
+          const f32x4 l4 = *reinterpret_cast<const f32x4*>(lse_s + mbq * 32 + i4 * 8 + kg * 4);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int i = i4 * 4 + r;
-            pr[i] = __builtin_amdgcn_exp2f(s[i] * c2 + tl[60 * mbq + 15 * i4 + r] - l4[r]);
-            if (sd.mixed && ((word >> (8 * i4 + r)) & 1u)) pr[i] = 0.0f;
-            ds[i] = pr[i] * (dp[i] - d4[r]);
-          }
+          for (int r = 0; r < 4; ++r) x[i4 * 4 + r] = s[i4 * 4 + r] * c2 + tl[60 * mbq + 15 * i4 + r] - l4[r];
+        }
+        if (sd.mixed) {  // wave-uniform
+          const uint32_t word = (uint32_t)(ap >> (32 * mbq));
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if ((word >> (8 * (i >> 2) + (i & 3))) & 1u) x[i] = -INFINITY;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          pr[i] = __builtin_amdgcn_exp2f(x[i]);
+          ds[i] = pr[i] * dp[i];
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
