@@ -592,7 +592,7 @@ int jg_bias_grad(void* gb, const void* g, int64_t batch, int64_t channels,
  *   w = sigmoid(lse - lse_acc); out_acc += w*(out - out_acc); lse_acc = logaddexp,
  * which is _online_softmax_merge_ (forward.py:23-61) without the round trip of
  * out_j through HBM; `out` / `lse` may then be NULL (bf16 and fp16 with d a multiple of 8
- * up to 128, fp32 with d = 32, 64 or 128; no bias, 16-byte aligned tensors, any sq and sk;
+ * up to 128, fp32 with d a multiple of 4 up to 128; no bias, 16-byte aligned tensors, any sq and sk;
  * JG_ERR_UNSUPPORTED otherwise).
  * Without a bias and with 16-byte aligned tensors those types and head sizes run on the
  * matrix cores (forward and backward). Everything else runs on one-thread-per-row kernels,
@@ -633,8 +633,8 @@ int jg_attn_bwd(void* dq, void* dk, void* dv, const void* dout, const void* q,
  * jg_attn_bwd returns for that chunk), dq the sum of the per-chunk dq, accumulated in fp32 and
  * rounded once (the reference adds the steps in q's dtype, backward.py:184, 269). k, v, dk, dv are
  * HOST arrays of n_chunks device pointers, read before the call returns. No bias.
- * Covered: bf16 and fp16, d a multiple of 8 up to 128, any lengths, 1 <= n_chunks <= 16, 16-byte aligned
- * tensors; JG_ERR_UNSUPPORTED otherwise (call jg_attn_bwd per chunk and add the dq). workspace as for
+ * Covered: bf16 and fp16, d a multiple of 8 up to 128, and fp32, d a multiple of 4 up to 128; any lengths,
+ * 1 <= n_chunks <= 16, 16-byte aligned tensors; JG_ERR_UNSUPPORTED otherwise (call jg_attn_bwd per chunk and add the dq). workspace as for
  * jg_attn_bwd. */
 int jg_attn_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q,
                        const void* const* k, const void* const* v, int64_t n_chunks, const void* out,

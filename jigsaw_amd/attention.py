@@ -101,7 +101,7 @@ def _bias_args(bias, batch, sq, sk):
 
 # --------------------------------------------------------------------------- #
 # The 16-bit matrix-core kernels take any lengths and any head size that is a multiple of 8 up to
-# 128, the fp32 ones any lengths at three head sizes, the one-thread-per-row kernels (bias, more
+# 128, the fp32 ones any lengths at multiples of 4 up to 128, the one-thread-per-row kernels (bias, more
 # batch entries than a grid dimension holds) a few head sizes. Other head sizes get zero columns:
 # they add nothing to the scores and give zero output columns, which are dropped. Narrow bf16 heads on
 # long sequences get them too, for the faster kernels of 64 columns (_as_64_columns).
@@ -118,10 +118,16 @@ def _mfma16(q, k, bias=None) -> bool:
             and max(q.shape[-2], k.shape[-2]) <= _MOST_ROWS and math.prod(q.shape[:-2]) <= _MOST_BATCH)
 
 
+def _mfma32(q, k) -> bool:
+    """Whether the fp32 matrix-core kernels take q against the keys k (their head size padded to a multiple of 4)."""
+    return (q.dtype == torch.float32 and q.shape[-1] <= 128 and max(q.shape[-2], k.shape[-2]) <= _MOST_ROWS
+            and math.prod(q.shape[:-2]) <= _MOST_BATCH)
+
+
 def _kernel_head_size(d: int, dtype=None, has_bias: bool = False) -> int:
     """Smallest head size the kernels beside the 16-bit matrix-core ones are built for that holds ``d`` columns;
-    ``d`` itself beyond the largest. fp32 without a bias goes to the sizes of its matrix-core kernels,
-    everything else to those of the one-thread-per-row kernels."""
+    ``d`` itself beyond the largest. fp32 without a bias goes to the widths of its matrix-core kernels,
+    everything else to the sizes of the one-thread-per-row kernels."""
     sizes = _F32_MFMA_HEAD_SIZES if dtype == torch.float32 and not has_bias else _KERNEL_HEAD_SIZES
     return next((n for n in sizes if n >= d), d)
 
@@ -147,6 +153,8 @@ def _as_64_columns(q, k, chunks: int = 1) -> bool:
 
 def _padded_head_size(q, k, bias) -> int:
     d = q.shape[-1]
+    if bias is None and _mfma32(q, k):
+        return (d + 3) // 4 * 4
     if not _mfma16(q, k, bias):
         return _kernel_head_size(d, q.dtype, bias is not None)
     return 64 if _as_64_columns(q, k) else (d + 7) // 8 * 8
@@ -257,14 +265,14 @@ def backward(grad_out, q, k, v, out, logsumexp, scale, *args, dropout_p=0.0, see
 # --------------------------------------------------------------------------- #
 def _fused_ok(q, k) -> bool:
     """Whether one launch attends the chunk AND merges into the running accumulators: the 16-bit matrix-core
-    kernels at head sizes that are multiples of 8, the fp32 one at head sizes 32 / 64 / 128 (any lengths,
+    kernels at head sizes that are multiples of 8, the fp32 one at multiples of 4 (any lengths,
     16-byte aligned tensors)."""
     d = q.shape[-1]
     if any(t.data_ptr() % 16 for t in (q, k)):
         return False
     if _as_64_columns(q, k):  # the merge is a kernel of its own then
         return False
-    return d in _F32_MFMA_HEAD_SIZES if q.dtype == torch.float32 else d % 8 == 0 and _mfma16(q, k)
+    return d % 4 == 0 and _mfma32(q, k) if q.dtype == torch.float32 else d % 8 == 0 and _mfma16(q, k)
 
 
 def attend_step_(q, kj, vj, scale, out, lse):
@@ -286,8 +294,8 @@ def attend_step_(q, kj, vj, scale, out, lse):
 def ring_forward(q, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.Tensor], scale, rank: int = 0):
     """``(out, lse)`` of one rank's queries over all P chunks, visited in ring order
     ``(rank + step) % P`` (forward_chunk_provider.py:190-192). The accumulator is
-    fp32 and cast to ``q.dtype`` once at the end (forward.py:160-167, 199). 16-bit chunks, all
-    resident here, go through one launch that keeps it in registers (a step's output is then not
+    fp32 and cast to ``q.dtype`` once at the end (forward.py:160-167, 199). Chunks that are all
+    resident here go through one launch that keeps it in registers (a step's output is then not
     rounded before it is merged, as it is step by step)."""
     P = len(k_chunks)
     order = [(rank + step) % P for step in range(P)]
@@ -309,7 +317,8 @@ _MAX_CHUNKS_PER_CALL = 16
 def _resident(q, k_chunks, v_chunks) -> bool:
     """Whether the one-pass kernels take q against these chunks."""
     k0 = k_chunks[0]
-    return (len(k_chunks) == len(v_chunks) <= _MAX_CHUNKS_PER_CALL and q.is_cuda and q.shape[-1] % 8 == 0 and _mfma16(q, k0)
+    covered = q.shape[-1] % 4 == 0 and _mfma32(q, k0) or q.shape[-1] % 8 == 0 and _mfma16(q, k0)
+    return (covered and len(k_chunks) == len(v_chunks) <= _MAX_CHUNKS_PER_CALL and q.is_cuda
             and k0.shape[:-2] == q.shape[:-2] and k0.shape[-1] == q.shape[-1]
             and all(t.shape == k0.shape and t.device == q.device for t in (*k_chunks, *v_chunks)))
 

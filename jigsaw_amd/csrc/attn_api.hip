@@ -22,13 +22,12 @@ int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
                          const void* const* k, const void* const* v, int nchunks, const void* out, const float* lse,
                          long long batch, int sq, int sk, float scale, void* ws, hipStream_t s);
 bool attn_wide_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias);
-bool attn_f32_mfma_fwd_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias);
-int attn_f32_mfma_fwd(void* out, float* lse, const void* q, const void* k, const void* v, long long batch, int sq,
-                      int sk, int d, float scale, float* out_acc, float* lse_acc, hipStream_t s);
-bool attn_f32_mfma_bwd_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias);
-int attn_f32_mfma_bwd(void* dq, void* dk, void* dv, const void* dout, const void* q, const void* k, const void* v,
-                      const void* out, const float* lse, long long batch, int sq, int sk, int d, float scale,
-                      void* workspace, hipStream_t s);
+bool attn_f32_mfma_supported(long long batch, int sq, int sk, int d, int chunks, int dtype, bool has_bias);
+int attn_f32_mfma_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v, int chunks,
+                             long long batch, int sq, int sk, int d, float scale, float* out_acc, float* lse_acc, hipStream_t s);
+int attn_f32_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q, const void* const* k,
+                             const void* const* v, int chunks, const void* out, const float* lse, long long batch, int sq, int sk,
+                             int d, float scale, void* workspace, hipStream_t s);
 bool attn_window_supported(long long batch, int sq, int sk, int d, int dtype);
 int attn_window_fwd(void* out, float* lse, const void* q, const void* k, const void* v,
                     long long batch, float scale, const float* bias, long long bias_period,
@@ -101,15 +100,15 @@ extern "C" int jg_attn_fwd(void* out, float* lse, const void* q, const void* k, 
       aligned16({out, q, k, v, out_acc}))
     return jg::attn_wide_fwd_chunks(out, lse, q, &k, &v, 1, batch, (int)sq, (int)sk, (int)d, dtype, scale, out_acc,
                                     lse_acc, s);
-  if (jg::attn_f32_mfma_fwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr) &&
+  if (jg::attn_f32_mfma_supported(batch, (int)sq, (int)sk, (int)d, 1, dtype, bias != nullptr) &&
       aligned16({out, q, k, v, out_acc}))
-    return jg::attn_f32_mfma_fwd(out, lse, q, k, v, batch, (int)sq, (int)sk, (int)d, scale, out_acc, lse_acc, s);
+    return jg::attn_f32_mfma_fwd_chunks(out, lse, q, &k, &v, 1, batch, (int)sq, (int)sk, (int)d, scale, out_acc, lse_acc, s);
   if (!jg::attn_generic_supported((int)d))
     JG_FAIL(JG_ERR_UNSUPPORTED, "%s: head size %lld not in {8, 16, 32, 64, 96, 128}", who, (long long)d);
   if (out_acc != nullptr)
     JG_FAIL(JG_ERR_UNSUPPORTED,
             "%s: the fused merge needs an MFMA path (bf16 or fp16 with d a multiple of 8 up to 128,"
-            " fp32 with d in {32, 64, 128}, no bias, 16-byte aligned tensors);"
+            " fp32 with d a multiple of 4 up to 128, no bias, 16-byte aligned tensors);"
             " call jg_lse_merge after the core instead", who);
   rc = jg::attn_generic_fwd(out, lse, q, k, v, batch, (int)sq, (int)sk, (int)d, scale, bias,
                             bias_period, dtype, s);
@@ -153,10 +152,10 @@ extern "C" int jg_attn_bwd(void* dq, void* dk, void* dv, const void* dout, const
       aligned16({dq, dk, dv, dout, q, k, v, out}))
     return jg::attn_wide_bwd_chunks(dq, &dk, &dv, dout, q, &k, &v, 1, out, lse, batch, (int)sq, (int)sk, (int)d,
                                     dtype, scale, workspace, s);
-  if (dbias == nullptr && jg::attn_f32_mfma_bwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, bias != nullptr) &&
+  if (dbias == nullptr && jg::attn_f32_mfma_supported(batch, (int)sq, (int)sk, (int)d, 1, dtype, bias != nullptr) &&
       aligned16({dq, dk, dv, dout, q, k, v, out}))
-    return jg::attn_f32_mfma_bwd(dq, dk, dv, dout, q, k, v, out, lse, batch, (int)sq, (int)sk, (int)d, scale,
-                                 workspace, s);
+    return jg::attn_f32_mfma_bwd_chunks(dq, &dk, &dv, dout, q, &k, &v, 1, out, lse, batch, (int)sq, (int)sk, (int)d, scale,
+                                        workspace, s);
   if (!jg::attn_generic_supported((int)d))
     JG_FAIL(JG_ERR_UNSUPPORTED, "%s: head size %lld not in {8, 16, 32, 64, 96, 128}", who, (long long)d);
   return jg::attn_generic_bwd(dq, dk, dv, static_cast<float*>(workspace), dbias, dout, q, k, v, out,
@@ -182,7 +181,9 @@ extern "C" int jg_attn_fwd_chunks(void* out, float* lse, const void* q, const vo
   if (aligned && jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, false))
     return jg::attn_wide_fwd_chunks(out, lse, q, k, v, (int)n_chunks, batch, (int)sq, (int)sk, (int)d, dtype, scale,
                                     nullptr, nullptr, s);
-  JG_FAIL(JG_ERR_UNSUPPORTED, "%s: bf16 or fp16, d a multiple of 8 up to 128, 16-byte aligned tensors", who);
+  if (aligned && jg::attn_f32_mfma_supported(batch, (int)sq, (int)sk, (int)d, (int)n_chunks, dtype, false))
+    return jg::attn_f32_mfma_fwd_chunks(out, lse, q, k, v, (int)n_chunks, batch, (int)sq, (int)sk, (int)d, scale, nullptr, nullptr, s);
+  JG_FAIL(JG_ERR_UNSUPPORTED, "%s: bf16 or fp16, d a multiple of 8 up to 128, or fp32, d a multiple of 4 up to 128; 16-byte aligned tensors", who);
 }
 
 extern "C" int jg_attn_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q,
@@ -208,5 +209,8 @@ extern "C" int jg_attn_bwd_chunks(void* dq, void* const* dk, void* const* dv, co
   if (aligned && jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, false))
     return jg::attn_wide_bwd_chunks(dq, dk, dv, dout, q, k, v, (int)n_chunks, out, lse, batch, (int)sq, (int)sk, (int)d,
                                     dtype, scale, workspace, s);
-  JG_FAIL(JG_ERR_UNSUPPORTED, "%s: bf16 or fp16, d a multiple of 8 up to 128, 16-byte aligned tensors", who);
+  if (aligned && jg::attn_f32_mfma_supported(batch, (int)sq, (int)sk, (int)d, (int)n_chunks, dtype, false))
+    return jg::attn_f32_mfma_bwd_chunks(dq, dk, dv, dout, q, k, v, (int)n_chunks, out, lse, batch, (int)sq, (int)sk, (int)d, scale,
+                                        workspace, s);
+  JG_FAIL(JG_ERR_UNSUPPORTED, "%s: bf16 or fp16, d a multiple of 8 up to 128, or fp32, d a multiple of 4 up to 128; 16-byte aligned tensors", who);
 }

@@ -1,8 +1,7 @@
 // fp32 attention core on the matrix cores (v_mfma_f32_32x32x2_f32): forward with the natural-log
-// LSE and, optionally, the merge into a running (out_acc, lse_acc) pair of a ring of chunks.
-// Any sequence lengths, head size 32, 64 or 128, no bias. fp32 inputs took the one-thread-per-row
-// kernels before (LDS broadcasts, 4 % of the fp32 peak); here a wavefront owns 32 queries and
-// walks the keys 32 at a time:
+// LSE and, optionally, the merge into a running (out_acc, lse_acc) pair of a ring of chunks; backward.
+// Any lengths, head sizes that are multiples of 4 up to 128, one or several K / V chunks a launch, no bias.
+// A wavefront owns 32 queries and walks the keys 32 at a time:
 //
 //   S^T = K Q^T      A = K (row = key), B = Q^T (column = query); the two contraction slots of an
 //                    MFMA step belong to the two halves of the wavefront, and half g owns the
@@ -13,10 +12,19 @@
 //   O^T = V^T P^T    A = V^T (row = head-size index), B = P^T: step i contracts the two keys whose
 //                    probabilities the two halves hold in element i, so P never moves.
 //
+// Workgroups of four wavefronts: R of them take 32 rows each of the resident side, and 4 / R groups of R
+// share the streamed tiles out among themselves, each with a tile of its own in LDS; their partial
+// results meet in LDS at the end. R = 4 reads the streamed side once for 128 rows; R = 1 gives a head of few
+// rows four times the workgroups, each a quarter as long, and leaves fewer wavefronts without rows.
+// The chunks of a ring are one launch: a launch a chunk held 90 workgroups at 45 heads x 171 tokens, and the
+// backward's four launches a chunk a fifth of its time.
+// D: the kernel's width, 32, 64, 96 or 128; a head size d below it (d % 4 == 0) has its missing columns as zeros
+// in LDS and registers and no copies in memory.
+//
 // Reference behaviour restated here:
 //   jigsaw/modules/attention/_functional/cores/math.py:69-78   (forward, lse = logsumexp of the scaled scores)
 //   jigsaw/modules/attention/_functional/forward.py (merge of a chunk into the running output by its LSE)
-#include "jg_common.h"
+#include "attn_chunks.h"
 
 namespace {
 
@@ -25,88 +33,181 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
-constexpr int kBQ = 32 * kWaves;  // queries per workgroup
-constexpr int kBK = 32;           // keys per step
-
-struct F32Params {
-  float* out;          // (batch, sq, D) or NULL
-  float* lse;          // (batch, sq) or NULL
-  const float* q;      // (batch, sq, D)
-  const float* k;      // (batch, sk, D)
-  const float* v;      // (batch, sk, D)
-  float* out_acc;      // (batch, sq, D) merged in place, or NULL
-  float* lse_acc;      // (batch, sq) merged in place, or NULL
-  int sq, sk, q_blocks;
-  float scale_log2;    // scale * log2(e)
-};
+constexpr int kBK = 32;  // rows of the streamed side per step
 
 // key row (inside a 32-key step) of accumulator element i in half g: the 32x32 result layout
 __device__ __forceinline__ int row_of(int i, int g) { return (i >> 2) * 8 + g * 4 + (i & 3); }
 
-template <int D>
-__global__ __launch_bounds__(kThreads) void attn_f32_mfma_fwd_kernel(F32Params p) {
-  constexpr int H = D / 2;        // contraction slots of one half
-  constexpr int PITCH = D + 4;    // LDS row pitch in floats: 16-byte rows, the b128 reads of 16 rows cover all banks
-  constexpr int PIECES = D / 32;  // 16-byte pieces of a 32 x D tile per thread
-  constexpr int NT = D / 32;      // 32-wide head-size tiles of the output
-  __shared__ float Ks[kBK * PITCH];
-  __shared__ float Vs[kBK * PITCH];
+template <int D, int R>
+struct Shape {
+  static constexpr int G = kWaves / R;            // groups that share the streamed tiles out
+  static constexpr int H = D / 2;                 // contraction slots of one half
+  static constexpr int PITCH = D + 4;             // LDS row pitch in floats: 16-byte rows, the b128 reads of 16 rows cover all banks
+  static constexpr int NT = D / 32;               // 32-wide head-size tiles
+  static constexpr int TG = 64 * R;               // threads of a group
+  static constexpr int PIECES = kBK * D / 4 / TG; // 16-byte pieces of a 32 x D tile per thread
+  static constexpr int TILE = kBK * PITCH;        // floats
+  static constexpr int GROUP = 2 * TILE + 2 * kBK;  // two tiles; 32 lse and 32 delta
+  static constexpr int LDS = G * GROUP * 4;
+};
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 5, n = lane & 31;
-  const long long b = blockIdx.x / p.q_blocks;
-  const int q0 = (int)(blockIdx.x % p.q_blocks) * kBQ;
-  const int qrow = q0 + wave * 32 + n;
-  const bool q_live = qrow < p.sq;
-  const float* kb_base = p.k + b * (long long)p.sk * D;
-  const float* vb_base = p.v + b * (long long)p.sk * D;
+template <int D, int R>
+using Pieces = f32x4[Shape<D, R>::PIECES];
 
-  // this lane's slice of its query, scaled
-  float qf[H];
-  {
-    const float* qp = p.q + (b * p.sq + (q_live ? qrow : p.sq - 1)) * (long long)D + g * H;
-#pragma unroll
-    for (int j = 0; j < H; j += 4) {
-      const f32x4 t = *reinterpret_cast<const f32x4*>(qp + j);
-      qf[j] = t.x * p.scale_log2;
-      qf[j + 1] = t.y * p.scale_log2;
-      qf[j + 2] = t.z * p.scale_log2;
-      qf[j + 3] = t.w * p.scale_log2;
+// Where a wavefront stands.
+template <int R>
+struct Seat {
+  int lane, g, n, group, row_wave, gt;
+  __device__ __forceinline__ Seat() {
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    lane = tid & 63;
+    g = lane >> 5;
+    n = lane & 31;
+    group = wave / R;
+    row_wave = wave % R;
+    gt = tid - group * 64 * R;
+  }
+};
+// Workgroups go to the 8 XCDs round-robin; each XCD gets a contiguous range, so that the workgroups of a head meet in one L2.
+__device__ __forceinline__ unsigned block_id() {
+  const unsigned total = gridDim.x, id = blockIdx.x;
+  return (total & 7u) == 0 ? (id & 7u) * (total >> 3) + (id >> 3) : id;
+}
+// The steps of a group: number group, group + G, ... of the chunks' steps in order.
+struct Walk {
+  int chunk, step, left;
+  __device__ __forceinline__ Walk(int group, int G, int per_chunk, int chunks) : chunk(0), step(group) {
+    const int total = per_chunk * chunks;
+    left = total > group ? (total - group + G - 1) / G : 0;
+    settle(per_chunk);
+  }
+  __device__ __forceinline__ void settle(int per_chunk) {
+    while (step >= per_chunk) {
+      step -= per_chunk;
+      ++chunk;
     }
   }
+  __device__ __forceinline__ void advance(int G, int per_chunk) {
+    step += G;
+    --left;
+    settle(per_chunk);
+  }
+};
 
-  f32x16 o[NT];
+// A 32 x D tile of two tensors into registers (rows past `rows` read the last row; those of the
+// second tensor become zero, and so do columns past d), and from there into LDS.
+template <int D, int R>
+__device__ __forceinline__ void fetch_tiles(Pieces<D, R>& a, Pieces<D, R>& b, const float* abase,
+                                            const float* bbase, int row0, int rows, int d, int gt) {
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int i = 0; i < Shape<D, R>::PIECES; ++i) {
+    const int e = gt + Shape<D, R>::TG * i, row = e / (D / 4), c = e % (D / 4) * 4;
+    const int r = row0 + row;
+    const bool there = c < d;
+    const long long at = (long long)(r < rows ? r : rows - 1) * d + (there ? c : 0);
+    const f32x4 t = *reinterpret_cast<const f32x4*>(abase + at), u = *reinterpret_cast<const f32x4*>(bbase + at);
+    a[i] = there ? t : zero;
+    b[i] = there && r < rows ? u : zero;
+  }
+}
+template <int D, int R>
+__device__ __forceinline__ void store_tiles(float* as, float* bs, const Pieces<D, R>& a, const Pieces<D, R>& b, int gt) {
+#pragma unroll
+  for (int i = 0; i < Shape<D, R>::PIECES; ++i) {
+    const int e = gt + Shape<D, R>::TG * i, row = e / (D / 4), c = e % (D / 4) * 4;
+    *reinterpret_cast<f32x4*>(as + row * (D + 4) + c) = a[i];
+    *reinterpret_cast<f32x4*>(bs + row * (D + 4) + c) = b[i];
+  }
+}
+// This lane's slice of a row (columns g D/2 ..), times mul.
+template <int D>
+__device__ __forceinline__ void load_slice(float (&f)[D / 2], const float* row, int g, int d, float mul) {
+#pragma unroll
+  for (int j = 0; j < D / 2; j += 4) {
+    const bool there = g * (D / 2) + j < d;
+    const f32x4 t = *reinterpret_cast<const f32x4*>(row + (there ? g * (D / 2) + j : 0));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[j + e] = there ? t[e] * mul : 0.0f;
+  }
+}
+// acc of the groups behind the first into LDS, and from there onto the first group's (the caller's barriers).
+template <int NT>
+__device__ __forceinline__ void put_acc(float* at, const f32x16 (&acc)[NT]) {
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) o[t][i] = 0.0f;
+    for (int i = 0; i < 16; ++i) at[(t * 16 + i) * 64] = acc[t][i];
+}
+template <int NT>
+__device__ __forceinline__ void add_acc(f32x16 (&acc)[NT], const float* at, float mul) {
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[t][i] += at[(t * 16 + i) * 64] * mul;
+}
+template <int NT>
+__device__ __forceinline__ void clear_acc(f32x16 (&acc)[NT]) {
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
+}
+
+struct F32Params {
+  const float* q;      // (batch, sq, d)
+  float* out;          // (batch, sq, d) or NULL
+  float* lse;          // (batch, sq) or NULL
+  float* out_acc;      // (batch, sq, d) merged in place, or NULL
+  float* lse_acc;      // (batch, sq) merged in place, or NULL
+  int sq, sk, d, chunks, blocks;  // blocks of 32 R queries of a batch entry
+  float scale_log2;    // scale * log2(e)
+};
+
+template <int D, int R>
+__global__ __launch_bounds__(kThreads) void attn_f32_mfma_fwd_kernel(jg::ChunkTable, F32Params p) {
+  typedef Shape<D, R> S;
+  constexpr int H = S::H, PITCH = S::PITCH, NT = S::NT, G = S::G;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  const Seat<R> me;
+  const int g = me.g, n = me.n;
+  float* Ks = smem + me.group * S::GROUP;
+  float* Vs = Ks + S::TILE;
+  const unsigned id = block_id();
+  const long long b = id / (unsigned)p.blocks;
+  const int wave_row = (int)(id % (unsigned)p.blocks) * (32 * R) + me.row_wave * 32;
+  const bool wave_live = wave_row < p.sq;  // uniform: a wavefront without rows only helps with the tiles
+  const int qrow = wave_row + n;
+  const bool q_live = qrow < p.sq;
+  const long long kv_at = b * (long long)p.sk * p.d;
+
+  float qf[H];  // this lane's slice of its query, scaled
+  load_slice<D>(qf, p.q + (b * p.sq + (q_live ? qrow : p.sq - 1)) * (long long)p.d, g, p.d, p.scale_log2);
+
+  f32x16 o[NT];
+  clear_acc(o);
   float m = -INFINITY, l = 0.0f;
 
-  const int steps = (p.sk + kBK - 1) / kBK;
-  f32x4 kreg[PIECES], vreg[PIECES];
-  auto fetch = [&](int step) {
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) {
-      const int e = tid + kThreads * i, row = e / (D / 4), c4 = e % (D / 4);
-      const int key = step * kBK + row;
-      const long long at = (long long)(key < p.sk ? key : p.sk - 1) * D + 4 * c4;
-      kreg[i] = *reinterpret_cast<const f32x4*>(kb_base + at);
-      const f32x4 t = *reinterpret_cast<const f32x4*>(vb_base + at);
-      const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-      vreg[i] = key < p.sk ? t : zero;  // a key past the end weighs 0; its V row must not be 0 * anything
-    }
+  const int per_chunk = (p.sk + kBK - 1) / kBK;
+  Walk w(me.group, G, per_chunk, p.chunks);
+  const int steps = (per_chunk * p.chunks + G - 1) / G;  // of the first group; the others have as many or one less
+  Pieces<D, R> kreg, vreg;
+  auto fetch = [&]() {
+    if (w.left > 0)
+      fetch_tiles<D, R>(kreg, vreg, reinterpret_cast<const float*>(jg::chunk_entry(0, w.chunk)) + kv_at,
+                        reinterpret_cast<const float*>(jg::chunk_entry(1, w.chunk)) + kv_at, w.step * kBK, p.sk, p.d, me.gt);
   };
-  fetch(0);
-  for (int step = 0; step < steps; ++step) {
+  fetch();
+  for (int it = 0; it < steps; ++it) {
+    const bool mine = w.left > 0;
+    const int key0 = w.step * kBK;
     __syncthreads();  // every wavefront is done with the previous tile
-#pragma unroll
-    for (int i = 0; i < PIECES; ++i) {
-      const int e = tid + kThreads * i, row = e / (D / 4), c4 = e % (D / 4);
-      *reinterpret_cast<f32x4*>(Ks + row * PITCH + 4 * c4) = kreg[i];
-      *reinterpret_cast<f32x4*>(Vs + row * PITCH + 4 * c4) = vreg[i];
-    }
+    if (mine) store_tiles<D, R>(Ks, Vs, kreg, vreg, me.gt);
     __syncthreads();
-    if (step + 1 < steps) fetch(step + 1);
+    if (!mine) continue;  // (the last iteration, groups behind the first)
+    w.advance(G, per_chunk);
+    fetch();
+    if (!wave_live) continue;
 
     // S^T[key][query], in units of log2
     f32x16 s;
@@ -120,10 +221,10 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_fwd_kernel(F32Params p
       s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qf[j + 2], s, 0, 0, 0);
       s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qf[j + 3], s, 0, 0, 0);
     }
-    if ((step + 1) * kBK > p.sk) {  // the last, ragged step
+    if (key0 + kBK > p.sk) {  // a chunk's last, ragged step
 #pragma unroll
       for (int i = 0; i < 16; ++i)
-        if (step * kBK + row_of(i, g) >= p.sk) s[i] = -INFINITY;
+        if (key0 + row_of(i, g) >= p.sk) s[i] = -INFINITY;
     }
     float mx = s[0];
 #pragma unroll
@@ -154,14 +255,41 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_fwd_kernel(F32Params p
     }
   }
 
+  if (G > 1) {  // the groups' results by their maxima, in the order of the groups
+    constexpr int PART = (NT * 16 + 2) * 64;
+    __syncthreads();
+    if (me.group > 0) {
+      float* at = smem + ((me.group - 1) * R + me.row_wave) * PART + me.lane;
+      put_acc(at, o);
+      at[NT * 16 * 64] = m;
+      at[(NT * 16 + 1) * 64] = l;
+    }
+    __syncthreads();
+    if (me.group > 0) return;
+#pragma unroll
+    for (int k = 1; k < G; ++k) {
+      const float* at = smem + ((k - 1) * R + me.row_wave) * PART + me.lane;
+      const float mk = at[NT * 16 * 64], lk = at[(NT * 16 + 1) * 64];
+      if (per_chunk * p.chunks <= k) break;  // a group that had no step
+      const float top = fmaxf(m, mk);
+      const float mine = __builtin_amdgcn_exp2f(m - top), other = __builtin_amdgcn_exp2f(mk - top);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[t][i] *= mine;
+      add_acc(o, at, other);
+      l = l * mine + lk * other;
+      m = top;
+    }
+  }
   if (!q_live) return;
   const float inv = 1.0f / l;
   const float lse_j = (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;  // v_log_f32 is log2
   const long long qi = b * p.sq + qrow;
-  float w = 0.0f;
+  float wt = 0.0f;
   if (p.out_acc != nullptr) {
     const float l_old = p.lse_acc[qi];
-    w = 1.0f / (1.0f + expf(l_old - lse_j));  // sigmoid(lse_j - l_old); l_old = -inf -> 1
+    wt = 1.0f / (1.0f + expf(l_old - lse_j));  // sigmoid(lse_j - l_old); l_old = -inf -> 1
     if (g == 0) p.lse_acc[qi] = fmaxf(l_old, lse_j) + log1pf(expf(-fabsf(l_old - lse_j)));
   }
   if (g == 0 && p.lse != nullptr) p.lse[qi] = lse_j;
@@ -169,15 +297,17 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_fwd_kernel(F32Params p
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
-      const long long at = qi * D + 32 * t + 8 * i4 + 4 * g;
+      const int c = 32 * t + 8 * i4 + 4 * g;
+      if (c >= p.d) continue;
+      const long long at = qi * p.d + c;
       f32x4 val = {o[t][4 * i4] * inv, o[t][4 * i4 + 1] * inv, o[t][4 * i4 + 2] * inv, o[t][4 * i4 + 3] * inv};
       if (p.out != nullptr) *reinterpret_cast<f32x4*>(p.out + at) = val;
       if (p.out_acc != nullptr) {
         f32x4 a = *reinterpret_cast<const f32x4*>(p.out_acc + at);
-        a.x += w * (val.x - a.x);
-        a.y += w * (val.y - a.y);
-        a.z += w * (val.z - a.z);
-        a.w += w * (val.w - a.w);
+        a.x += wt * (val.x - a.x);
+        a.y += wt * (val.y - a.y);
+        a.z += wt * (val.z - a.z);
+        a.w += wt * (val.w - a.w);
         *reinterpret_cast<f32x4*>(p.out_acc + at) = a;
       }
     }
@@ -188,114 +318,89 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_fwd_kernel(F32Params p
 // P = exp(S - lse), dS = P * (dO V^T - delta), dQ = scale dS K, dK = scale dS^T Q, dV = P^T dO.
 // Two kernels with the forward's operand placement. attn_f32_mfma_dq_kernel: a wavefront owns 32
 // queries (a lane: one query, 16 keys a step), S^T = K Q^T and dP^T = V dO^T with the Q and dO
-// slices in registers, then dQ^T += K^T dS^T with dS^T as it lies in the registers.
-// attn_f32_mfma_dkv_kernel: a wavefront owns 32 keys (a lane: one key, 16 queries a step),
-// S = Q K^T and dP = dO V^T with the K and V slices in registers, then dV^T += dO^T P and
+// slices in registers, then dQ^T += K^T dS^T with dS^T as it lies in the registers, over all chunks; it
+// leaves delta for the other. attn_f32_mfma_dkv_kernel: a wavefront owns 32 keys (a lane: one key, 16 queries a
+// step) of one chunk, S = Q K^T and dP = dO V^T with the K and V slices in registers, then dV^T += dO^T P and
 // dK^T += Q^T dS. Both recompute S and dP (6 + 8 matrix products of 32 x 32 x D per tile pair for
 // the 5 the mathematics needs once).
 struct F32BwdParams {
-  float* dq;           // (batch, sq, D)
-  float* dk;           // (batch, sk, D)
-  float* dv;           // (batch, sk, D)
-  const float* dout;   // (batch, sq, D)
+  float* dq;           // (batch, sq, d)
+  const float* dout;   // (batch, sq, d)
   const float* q;
-  const float* k;
-  const float* v;
+  const float* out;
   const float* lse;    // (batch, sq) natural log
-  const float* delta;  // (batch, sq)
-  int sq, sk, blocks_per_batch;
+  float* delta;        // (batch, sq)
+  int sq, sk, d, chunks, blocks;  // blocks of 32 R resident rows
   float scale, scale_log2;
 };
 
-template <int D>
-__global__ __launch_bounds__(kThreads) void attn_f32_delta_kernel(float* __restrict__ delta,
-                                                                  const float* __restrict__ dout,
-                                                                  const float* __restrict__ out, long long rows) {
-  const long long r = (long long)blockIdx.x * (kThreads / 16) + threadIdx.x / 16;
-  const int sl = threadIdx.x & 15;
-  float a = 0.0f;
-  if (r < rows) {
-    for (int c = sl * 4; c < D; c += 64) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(dout + r * D + c);
-      const f32x4 y = *reinterpret_cast<const f32x4*>(out + r * D + c);
-      a += x.x * y.x + x.y * y.y + x.z * y.z + x.w * y.w;
-    }
-  }
-  for (int o = 8; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
-  if (r < rows && sl == 0) delta[r] = a;
-}
-
-// A 32 x D tile of two tensors into registers (rows past `rows` read the last row; those of the
-// second tensor become zero), and from there into LDS.
-template <int D>
-__device__ __forceinline__ void fetch_tiles(f32x4 (&a)[D / 32], f32x4 (&b)[D / 32], const float* abase,
-                                            const float* bbase, int row0, int rows, int tid) {
-#pragma unroll
-  for (int i = 0; i < D / 32; ++i) {
-    const int e = tid + kThreads * i, row = e / (D / 4), c4 = e % (D / 4);
-    const int r = row0 + row;
-    const long long at = (long long)(r < rows ? r : rows - 1) * D + 4 * c4;
-    a[i] = *reinterpret_cast<const f32x4*>(abase + at);
-    const f32x4 t = *reinterpret_cast<const f32x4*>(bbase + at);
-    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    b[i] = r < rows ? t : zero;
-  }
-}
-template <int D>
-__device__ __forceinline__ void store_tiles(float* as, float* bs, const f32x4 (&a)[D / 32], const f32x4 (&b)[D / 32],
-                                            int tid) {
-#pragma unroll
-  for (int i = 0; i < D / 32; ++i) {
-    const int e = tid + kThreads * i, row = e / (D / 4), c4 = e % (D / 4);
-    *reinterpret_cast<f32x4*>(as + row * (D + 4) + 4 * c4) = a[i];
-    *reinterpret_cast<f32x4*>(bs + row * (D + 4) + 4 * c4) = b[i];
-  }
-}
-
-template <int D>
-__global__ __launch_bounds__(kThreads) void attn_f32_mfma_dq_kernel(F32BwdParams p) {
-  constexpr int H = D / 2, PITCH = D + 4, NT = D / 32;
-  __shared__ float Ks[kBK * PITCH];
-  __shared__ float Vs[kBK * PITCH];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 5, n = lane & 31;
-  const long long b = blockIdx.x / p.blocks_per_batch;
-  const int qrow = (int)(blockIdx.x % p.blocks_per_batch) * kBQ + wave * 32 + n;
-  const bool q_live = qrow < p.sq;
-  const long long qi = b * p.sq + (q_live ? qrow : p.sq - 1);
-  const float* kb_base = p.k + b * (long long)p.sk * D;
-  const float* vb_base = p.v + b * (long long)p.sk * D;
-
-  float qf[H], dof[H];
-#pragma unroll
-  for (int j = 0; j < H; j += 4) {
-    const f32x4 t = *reinterpret_cast<const f32x4*>(p.q + qi * D + g * H + j);
-    const f32x4 u = *reinterpret_cast<const f32x4*>(p.dout + qi * D + g * H + j);
-    qf[j] = t.x * p.scale_log2;
-    qf[j + 1] = t.y * p.scale_log2;
-    qf[j + 2] = t.z * p.scale_log2;
-    qf[j + 3] = t.w * p.scale_log2;
-    dof[j] = u.x;
-    dof[j + 1] = u.y;
-    dof[j + 2] = u.z;
-    dof[j + 3] = u.w;
-  }
-  const float lse2 = p.lse[qi] * 1.4426950408889634f, dl = p.delta[qi];
-
-  f32x16 dq[NT];
+template <int D, int NT>
+__device__ __forceinline__ void store_rows(float* row, const f32x16 (&acc)[NT], int g, int d, float mul) {
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) dq[t][i] = 0.0f;
+    for (int i4 = 0; i4 < 4; ++i4) {
+      const int c = 32 * t + 8 * i4 + 4 * g;
+      if (c >= d) continue;
+      const f32x4 val = {acc[t][4 * i4] * mul, acc[t][4 * i4 + 1] * mul, acc[t][4 * i4 + 2] * mul, acc[t][4 * i4 + 3] * mul};
+      *reinterpret_cast<f32x4*>(row + c) = val;
+    }
+}
 
-  const int steps = (p.sk + kBK - 1) / kBK;
-  f32x4 kreg[NT], vreg[NT];
-  fetch_tiles<D>(kreg, vreg, kb_base, vb_base, 0, p.sk, tid);
-  for (int step = 0; step < steps; ++step) {
+template <int D, int R>
+__global__ __launch_bounds__(kThreads) void attn_f32_mfma_dq_kernel(jg::ChunkTable, F32BwdParams p) {
+  typedef Shape<D, R> S;
+  constexpr int H = S::H, PITCH = S::PITCH, NT = S::NT, G = S::G;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  const Seat<R> me;
+  const int g = me.g, n = me.n;
+  float* Ks = smem + me.group * S::GROUP;
+  float* Vs = Ks + S::TILE;
+  const unsigned id = block_id();
+  const long long b = id / (unsigned)p.blocks;
+  const int wave_row = (int)(id % (unsigned)p.blocks) * (32 * R) + me.row_wave * 32;
+  const bool wave_live = wave_row < p.sq;
+  const int qrow = wave_row + n;
+  const bool q_live = qrow < p.sq;
+  const long long qi = b * p.sq + (q_live ? qrow : p.sq - 1);
+  const long long kv_at = b * (long long)p.sk * p.d;
+
+  float qf[H], dof[H];
+  load_slice<D>(qf, p.q + qi * p.d, g, p.d, p.scale_log2);
+  load_slice<D>(dof, p.dout + qi * p.d, g, p.d, 1.0f);
+  const float lse2 = p.lse[qi] * 1.4426950408889634f;
+  float dl = 0.0f;
+#pragma unroll
+  for (int j = 0; j < H; j += 4) {
+    const bool there = g * H + j < p.d;
+    const f32x4 t = *reinterpret_cast<const f32x4*>(p.out + qi * p.d + (there ? g * H + j : 0));
+    if (there) dl += dof[j] * t.x + dof[j + 1] * t.y + dof[j + 2] * t.z + dof[j + 3] * t.w;
+  }
+  dl += __shfl_xor(dl, 32, 64);
+  if (me.group == 0 && g == 0 && q_live) p.delta[qi] = dl;
+
+  f32x16 dq[NT];
+  clear_acc(dq);
+  const int per_chunk = (p.sk + kBK - 1) / kBK;
+  Walk w(me.group, G, per_chunk, p.chunks);
+  const int steps = (per_chunk * p.chunks + G - 1) / G;
+  Pieces<D, R> kreg, vreg;
+  auto fetch = [&]() {
+    if (w.left > 0)
+      fetch_tiles<D, R>(kreg, vreg, reinterpret_cast<const float*>(jg::chunk_entry(0, w.chunk)) + kv_at,
+                        reinterpret_cast<const float*>(jg::chunk_entry(1, w.chunk)) + kv_at, w.step * kBK, p.sk, p.d, me.gt);
+  };
+  fetch();
+  for (int it = 0; it < steps; ++it) {
+    const bool mine = w.left > 0;
+    const int key0 = w.step * kBK;
     __syncthreads();
-    store_tiles<D>(Ks, Vs, kreg, vreg, tid);
+    if (mine) store_tiles<D, R>(Ks, Vs, kreg, vreg, me.gt);
     __syncthreads();
-    if (step + 1 < steps) fetch_tiles<D>(kreg, vreg, kb_base, vb_base, (step + 1) * kBK, p.sk, tid);
+    if (!mine) continue;
+    w.advance(G, per_chunk);
+    fetch();
+    if (!wave_live) continue;
 
     f32x16 s, dp;
 #pragma unroll
@@ -316,11 +421,11 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_dq_kernel(F32BwdParams
       s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qf[j + 3], s, 0, 0, 0);
       dp = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.w, dof[j + 3], dp, 0, 0, 0);
     }
-    const bool ragged = (step + 1) * kBK > p.sk;
+    const bool ragged = key0 + kBK > p.sk;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       float pr = __builtin_amdgcn_exp2f(s[i] - lse2);
-      if (ragged && step * kBK + row_of(i, g) >= p.sk) pr = 0.0f;
+      if (ragged && key0 + row_of(i, g) >= p.sk) pr = 0.0f;
       s[i] = pr * (dp[i] - dl);  // dS^T
     }
 #pragma unroll
@@ -330,82 +435,81 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_dq_kernel(F32BwdParams
       for (int t = 0; t < NT; ++t) dq[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(krow[32 * t], s[i], dq[t], 0, 0, 0);
     }
   }
-  if (!q_live) return;
+  if (G > 1) {
+    constexpr int PART = NT * 16 * 64;
+    __syncthreads();
+    if (me.group > 0) put_acc(smem + ((me.group - 1) * R + me.row_wave) * PART + me.lane, dq);
+    __syncthreads();
+    if (me.group > 0) return;
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const f32x4 val = {dq[t][4 * i4] * p.scale, dq[t][4 * i4 + 1] * p.scale, dq[t][4 * i4 + 2] * p.scale,
-                         dq[t][4 * i4 + 3] * p.scale};
-      *reinterpret_cast<f32x4*>(p.dq + qi * D + 32 * t + 8 * i4 + 4 * g) = val;
-    }
+    for (int k = 1; k < G; ++k) add_acc(dq, smem + ((k - 1) * R + me.row_wave) * PART + me.lane, 1.0f);
+  }
+  if (q_live) store_rows<D>(p.dq + qi * p.d, dq, g, p.d, p.scale);
 }
 
-template <int D>
-__global__ __launch_bounds__(kThreads) void attn_f32_mfma_dkv_kernel(F32BwdParams p) {
-  constexpr int H = D / 2, PITCH = D + 4, NT = D / 32;
-  __shared__ float Qs[kBK * PITCH];
-  __shared__ float dOs[kBK * PITCH];
-  __shared__ float lse2s[kBK];
-  __shared__ float deltas[kBK];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = lane >> 5, n = lane & 31;
-  const long long b = blockIdx.x / p.blocks_per_batch;
-  const int krow = (int)(blockIdx.x % p.blocks_per_batch) * kBQ + wave * 32 + n;
+template <int D, int R>
+__global__ __launch_bounds__(kThreads) void attn_f32_mfma_dkv_kernel(jg::ChunkTable, F32BwdParams p) {
+  typedef Shape<D, R> S;
+  constexpr int H = S::H, PITCH = S::PITCH, NT = S::NT, G = S::G;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  const Seat<R> me;
+  const int g = me.g, n = me.n;
+  float* Qs = smem + me.group * S::GROUP;
+  float* dOs = Qs + S::TILE;
+  float* lse2s = dOs + S::TILE;
+  float* deltas = lse2s + kBK;
+  const unsigned id = block_id(), per_entry = (unsigned)p.blocks * (unsigned)p.chunks;
+  const long long b = id / per_entry;
+  const int chunk = __builtin_amdgcn_readfirstlane((int)(id % per_entry / (unsigned)p.blocks));
+  const int wave_row = (int)(id % (unsigned)p.blocks) * (32 * R) + me.row_wave * 32;
+  const bool wave_live = wave_row < p.sk;
+  const int krow = wave_row + n;
   const bool k_live = krow < p.sk;
   const long long ki = b * p.sk + (k_live ? krow : p.sk - 1);
-  const float* qb_base = p.q + b * (long long)p.sq * D;
-  const float* dob_base = p.dout + b * (long long)p.sq * D;
+  const float* qb_base = p.q + b * (long long)p.sq * p.d;
+  const float* dob_base = p.dout + b * (long long)p.sq * p.d;
   const float* lse_base = p.lse + b * (long long)p.sq;
   const float* delta_base = p.delta + b * (long long)p.sq;
 
   float kf[H], vf[H];
-#pragma unroll
-  for (int j = 0; j < H; j += 4) {
-    const f32x4 t = *reinterpret_cast<const f32x4*>(p.k + ki * D + g * H + j);
-    const f32x4 u = *reinterpret_cast<const f32x4*>(p.v + ki * D + g * H + j);
-    kf[j] = t.x * p.scale_log2;
-    kf[j + 1] = t.y * p.scale_log2;
-    kf[j + 2] = t.z * p.scale_log2;
-    kf[j + 3] = t.w * p.scale_log2;
-    vf[j] = u.x;
-    vf[j + 1] = u.y;
-    vf[j + 2] = u.z;
-    vf[j + 3] = u.w;
-  }
+  load_slice<D>(kf, reinterpret_cast<const float*>(jg::chunk_entry(0, chunk)) + ki * p.d, g, p.d, p.scale_log2);
+  load_slice<D>(vf, reinterpret_cast<const float*>(jg::chunk_entry(1, chunk)) + ki * p.d, g, p.d, 1.0f);
   f32x16 dk[NT], dv[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      dk[t][i] = 0.0f;
-      dv[t][i] = 0.0f;
-    }
+  clear_acc(dk);
+  clear_acc(dv);
 
-  const int steps = (p.sq + kBK - 1) / kBK;
-  f32x4 qreg[NT], doreg[NT];
+  const int per_chunk = (p.sq + kBK - 1) / kBK;  // here the steps run over the queries, once
+  Walk w(me.group, G, per_chunk, 1);
+  const int steps = (per_chunk + G - 1) / G;
+  Pieces<D, R> qreg, doreg;
   float lreg = 0.0f, dreg = 0.0f;
-  auto fetch_rows = [&](int step) {  // the 32 queries' lse (in log2 units) and delta; 0 past the end
-    if (tid < kBK) {
-      const int r = step * kBK + tid;
+  auto fetch = [&]() {
+    if (w.left <= 0) return;
+    fetch_tiles<D, R>(qreg, doreg, qb_base, dob_base, w.step * kBK, p.sq, p.d, me.gt);
+    if (me.gt < kBK) {  // the 32 queries' lse (in log2 units) and delta; 0 past the end
+      const int r = w.step * kBK + me.gt;
       lreg = r < p.sq ? lse_base[r] * 1.4426950408889634f : 0.0f;
       dreg = r < p.sq ? delta_base[r] : 0.0f;
     }
   };
-  fetch_tiles<D>(qreg, doreg, qb_base, dob_base, 0, p.sq, tid);
-  fetch_rows(0);
-  for (int step = 0; step < steps; ++step) {
+  fetch();
+  for (int it = 0; it < steps; ++it) {
+    const bool mine = w.left > 0;
+    const int q0 = w.step * kBK;
     __syncthreads();
-    store_tiles<D>(Qs, dOs, qreg, doreg, tid);
-    if (tid < kBK) {
-      lse2s[tid] = lreg;
-      deltas[tid] = dreg;
+    if (mine) {
+      store_tiles<D, R>(Qs, dOs, qreg, doreg, me.gt);
+      if (me.gt < kBK) {
+        lse2s[me.gt] = lreg;
+        deltas[me.gt] = dreg;
+      }
     }
     __syncthreads();
-    if (step + 1 < steps) {
-      fetch_tiles<D>(qreg, doreg, qb_base, dob_base, (step + 1) * kBK, p.sq, tid);
-      fetch_rows(step + 1);
-    }
+    if (!mine) continue;
+    w.step += G;
+    --w.left;
+    fetch();
+    if (!wave_live) continue;
 
     f32x16 s, dp;
 #pragma unroll
@@ -426,12 +530,12 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_dkv_kernel(F32BwdParam
       s = __builtin_amdgcn_mfma_f32_32x32x2f32(qv.w, kf[j + 3], s, 0, 0, 0);
       dp = __builtin_amdgcn_mfma_f32_32x32x2f32(gv.w, vf[j + 3], dp, 0, 0, 0);
     }
-    const bool ragged = (step + 1) * kBK > p.sq;
+    const bool ragged = q0 + kBK > p.sq;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int qr = row_of(i, g);
       float pr = __builtin_amdgcn_exp2f(s[i] - lse2s[qr]);
-      if (ragged && step * kBK + qr >= p.sq) pr = 0.0f;
+      if (ragged && q0 + qr >= p.sq) pr = 0.0f;
       s[i] = pr;                          // P
       dp[i] = pr * (dp[i] - deltas[qr]);  // dS
     }
@@ -446,100 +550,135 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_dkv_kernel(F32BwdParam
       }
     }
   }
-  if (!k_live) return;
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const long long at = ki * D + 32 * t + 8 * i4 + 4 * g;
-      const f32x4 a = {dk[t][4 * i4] * p.scale, dk[t][4 * i4 + 1] * p.scale, dk[t][4 * i4 + 2] * p.scale,
-                       dk[t][4 * i4 + 3] * p.scale};
-      const f32x4 c = {dv[t][4 * i4], dv[t][4 * i4 + 1], dv[t][4 * i4 + 2], dv[t][4 * i4 + 3]};
-      *reinterpret_cast<f32x4*>(p.dk + at) = a;
-      *reinterpret_cast<f32x4*>(p.dv + at) = c;
+  if (G > 1) {
+    constexpr int PART = 2 * NT * 16 * 64;
+    __syncthreads();
+    if (me.group > 0) {
+      float* at = smem + ((me.group - 1) * R + me.row_wave) * PART + me.lane;
+      put_acc(at, dk);
+      put_acc(at + NT * 16 * 64, dv);
     }
+    __syncthreads();
+    if (me.group > 0) return;
+#pragma unroll
+    for (int k = 1; k < G; ++k) {
+      const float* at = smem + ((k - 1) * R + me.row_wave) * PART + me.lane;
+      add_acc(dk, at, 1.0f);
+      add_acc(dv, at + NT * 16 * 64, 1.0f);
+    }
+  }
+  if (!k_live) return;
+  store_rows<D>(reinterpret_cast<float*>(const_cast<char*>(jg::chunk_entry(2, chunk))) + ki * p.d, dk, g, p.d, p.scale);
+  store_rows<D>(reinterpret_cast<float*>(const_cast<char*>(jg::chunk_entry(3, chunk))) + ki * p.d, dv, g, p.d, 1.0f);
 }
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
+
+// Resident rows of a workgroup, in wavefronts: what the busiest compute unit has to do (its workgroups, each R / 4 of the
+// streamed side long, whether they run beside each other or in turn), a little more where the streamed side is read more often,
+// a little less at 32 columns, where several workgroups of one wavefront's tiles fit a compute unit. Forward / dQ / dK and dV, us,
+// one against two wavefronts of rows where both leave two units of work: 45 x 171 x 6 chunks at 32 34 / 45 / - and 39 / 50 / -, 16 x 700 x 4 at
+// 64 126 / 208 and 141 / 183, 24 x 350 x 5 at 80 178 / 223 and 119 / 157, 12 x 800 x 3 at 96 302 / 364 and 165 / 219. Whole steps before (a
+// launch a chunk of 128 rows each, 80 and 96 columns as 128 with copies) and now: 322 -> 121, 1061 -> 490, 1707 -> 435, 1960 -> 576;
+// launches that filled the chip 1963 -> 1875 (64 x 1000 x 3 at 64: 0.09 PFLOP/s of the matrix cores' 0.16) and 5410 -> 4860 (48 x 900 x 4 at 128).
+int width(long long rows, long long entries, int d, int least) {
+  int best = 4;
+  long long best_cost = -1;
+  for (int r = 4; r >= least; r /= 2) {
+    const long long cost = jg::cdiv(jg::cdiv(rows, 32 * r) * entries, jg::cu_count()) * (long long)r * (d <= 32 ? (r == 1 ? 97 : 100) : r == 4 ? 100 : r == 2 ? 103 : 110);
+    if (best_cost < 0 || cost < best_cost) {
+      best = r;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+// kernel<D, R><<<>>> for run-time d and R
+#define JG_F32_LAUNCH(KERNEL, DD, RR, BLOCKS, ...)                                                                             \
+  do {                                                                                                                         \
+    typedef Shape<DD, RR> S_;                                                                                                  \
+    if (S_::LDS > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(&KERNEL<DD, RR>),                                 \
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, S_::LDS) != hipSuccess)             \
+      JG_FAIL(JG_ERR_LAUNCH, "jg_attn(fp32 mfma): cannot reserve %d bytes of LDS", S_::LDS);                                   \
+    KERNEL<DD, RR><<<(unsigned)(BLOCKS), kThreads, S_::LDS, s>>>(__VA_ARGS__);                                                 \
+  } while (0)
+#define JG_F32_WIDTHS(KERNEL, DD, R, BLOCKS, ...)                              \
+  do {                                                                         \
+    if (R == 1) JG_F32_LAUNCH(KERNEL, DD, 1, BLOCKS, __VA_ARGS__);             \
+    else if (R == 2) JG_F32_LAUNCH(KERNEL, DD, 2, BLOCKS, __VA_ARGS__);        \
+    else JG_F32_LAUNCH(KERNEL, DD, 4, BLOCKS, __VA_ARGS__);                    \
+  } while (0)
+#define JG_F32_GO(KERNEL, D, R, BLOCKS, ...)                                   \
+  do {                                                                         \
+    if (D <= 32) JG_F32_WIDTHS(KERNEL, 32, R, BLOCKS, __VA_ARGS__);            \
+    else if (D <= 64) JG_F32_WIDTHS(KERNEL, 64, R, BLOCKS, __VA_ARGS__);       \
+    else if (D <= 96) JG_F32_WIDTHS(KERNEL, 96, R, BLOCKS, __VA_ARGS__);       \
+    else JG_F32_WIDTHS(KERNEL, 128, R, BLOCKS, __VA_ARGS__);                   \
+  } while (0)
 
 }  // namespace
 
 namespace jg {
 
-bool attn_f32_mfma_fwd_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias) {
+bool attn_f32_mfma_supported(long long batch, int sq, int sk, int d, int chunks, int dtype, bool has_bias) {
   if (dtype != JG_F32 || has_bias || batch <= 0 || sq <= 0 || sk <= 0) return false;
-  if (d != 32 && d != 64 && d != 128) return false;
-  const long long blocks = batch * ((sq + kBQ - 1) / kBQ);
-  return blocks <= 0x7fffffffLL;
+  if (d < 4 || d > 128 || d % 4 != 0) return false;
+  // workgroups of 32 rows, and the steps of all chunks, in 31 bits
+  return batch < (1ll << 31) && batch * cdiv((long long)sq, 32ll) < (1ll << 31) && batch * chunks * cdiv((long long)sk, 32ll) < (1ll << 31);
 }
 
-int attn_f32_mfma_fwd(void* out, float* lse, const void* q, const void* k, const void* v, long long batch, int sq,
-                      int sk, int d, float scale, float* out_acc, float* lse_acc, hipStream_t s) {
-  for (const void* ptr : {static_cast<const void*>(out), q, k, v, static_cast<const void*>(out_acc)})
+int attn_f32_mfma_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v, int chunks,
+                             long long batch, int sq, int sk, int d, float scale, float* out_acc, float* lse_acc, hipStream_t s) {
+  for (const void* ptr : {static_cast<const void*>(out), q, static_cast<const void*>(out_acc)})
     JG_REQUIRE(aligned16(ptr), "jg_attn_fwd: the fp32 matrix-core kernel needs 16-byte aligned tensors");
-  F32Params p;
+  const ChunkTable tab = chunk_table(k, v, nullptr, nullptr, chunks);
+  const int r = width(sq, batch, d, 1);
+  F32Params p = {};
+  p.q = static_cast<const float*>(q);
   p.out = static_cast<float*>(out);
   p.lse = lse;
-  p.q = static_cast<const float*>(q);
-  p.k = static_cast<const float*>(k);
-  p.v = static_cast<const float*>(v);
   p.out_acc = out_acc;
   p.lse_acc = lse_acc;
   p.sq = sq;
   p.sk = sk;
-  p.q_blocks = (sq + kBQ - 1) / kBQ;
+  p.d = d;
+  p.chunks = chunks;
+  p.blocks = (int)cdiv((long long)sq, 32ll * r);
   p.scale_log2 = scale * 1.4426950408889634f;
-  const unsigned blocks = (unsigned)(batch * p.q_blocks);
-  if (d == 32) attn_f32_mfma_fwd_kernel<32><<<blocks, kThreads, 0, s>>>(p);
-  else if (d == 64) attn_f32_mfma_fwd_kernel<64><<<blocks, kThreads, 0, s>>>(p);
-  else attn_f32_mfma_fwd_kernel<128><<<blocks, kThreads, 0, s>>>(p);
+  JG_F32_GO(attn_f32_mfma_fwd_kernel, d, r, batch * p.blocks, tab, p);
   JG_CHECK_LAUNCH("jg_attn_fwd(fp32 mfma)");
   return JG_OK;
 }
 
-bool attn_f32_mfma_bwd_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias) {
-  if (!attn_f32_mfma_fwd_supported(batch, sq, sk, d, dtype, has_bias)) return false;
-  return batch * ((sk + kBQ - 1) / kBQ) <= 0x7fffffffLL;
-}
-
 // workspace: (batch, sq) floats for delta
-int attn_f32_mfma_bwd(void* dq, void* dk, void* dv, const void* dout, const void* q, const void* k, const void* v,
-                      const void* out, const float* lse, long long batch, int sq, int sk, int d, float scale,
-                      void* workspace, hipStream_t s) {
-  for (const void* ptr : {static_cast<const void*>(dq), static_cast<const void*>(dk), static_cast<const void*>(dv),
-                          dout, q, k, v, out})
+int attn_f32_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q, const void* const* k,
+                             const void* const* v, int chunks, const void* out, const float* lse, long long batch, int sq, int sk,
+                             int d, float scale, void* workspace, hipStream_t s) {
+  for (const void* ptr : {static_cast<const void*>(dq), dout, q, out})
     JG_REQUIRE(aligned16(ptr), "jg_attn_bwd: the fp32 matrix-core kernels need 16-byte aligned tensors");
-  F32BwdParams p;
+  const ChunkTable tab = chunk_table(k, v, dk, dv, chunks);
+  F32BwdParams p = {};
   p.dq = static_cast<float*>(dq);
-  p.dk = static_cast<float*>(dk);
-  p.dv = static_cast<float*>(dv);
   p.dout = static_cast<const float*>(dout);
   p.q = static_cast<const float*>(q);
-  p.k = static_cast<const float*>(k);
-  p.v = static_cast<const float*>(v);
+  p.out = static_cast<const float*>(out);
   p.lse = lse;
-  float* delta = static_cast<float*>(workspace);
-  p.delta = delta;
+  p.delta = static_cast<float*>(workspace);
   p.sq = sq;
   p.sk = sk;
+  p.d = d;
+  p.chunks = chunks;
   p.scale = scale;
   p.scale_log2 = scale * 1.4426950408889634f;
-  const long long rows = batch * sq;
-  const unsigned delta_blocks = (unsigned)((rows + kThreads / 16 - 1) / (kThreads / 16));
-  const unsigned q_blocks = (unsigned)(batch * ((sq + kBQ - 1) / kBQ)), k_blocks = (unsigned)(batch * ((sk + kBQ - 1) / kBQ));
-#define JG_GO(DD)                                                                                          \
-  do {                                                                                                     \
-    attn_f32_delta_kernel<DD><<<delta_blocks, kThreads, 0, s>>>(delta, p.dout, static_cast<const float*>(out), rows); \
-    p.blocks_per_batch = (sq + kBQ - 1) / kBQ;                                                             \
-    attn_f32_mfma_dq_kernel<DD><<<q_blocks, kThreads, 0, s>>>(p);                                          \
-    p.blocks_per_batch = (sk + kBQ - 1) / kBQ;                                                             \
-    attn_f32_mfma_dkv_kernel<DD><<<k_blocks, kThreads, 0, s>>>(p);                                         \
-  } while (0)
-  if (d == 32) JG_GO(32);
-  else if (d == 64) JG_GO(64);
-  else JG_GO(128);
-#undef JG_GO
-  JG_CHECK_LAUNCH("jg_attn_bwd(fp32 mfma)");
+  // (dK / dV at 128 columns: no registers for tiles that one wavefront fetches alone)
+  const int rq = width(sq, batch, d, 1), rk = width(sk, batch * chunks, d, d > 96 ? 2 : 1);
+  p.blocks = (int)cdiv((long long)sq, 32ll * rq);
+  JG_F32_GO(attn_f32_mfma_dq_kernel, d, rq, batch * p.blocks, tab, p);
+  JG_CHECK_LAUNCH("jg_attn_bwd(fp32 mfma dq)");
+  p.blocks = (int)cdiv((long long)sk, 32ll * rk);
+  JG_F32_GO(attn_f32_mfma_dkv_kernel, d, rk, batch * chunks * p.blocks, tab, p);
+  JG_CHECK_LAUNCH("jg_attn_bwd(fp32 mfma dk dv)");
   return JG_OK;
 }
 

@@ -383,6 +383,36 @@ def test_backward_over_chunks_declines_what_it_does_not_cover(dev):
     assert ja.backward_chunks(qb, qb, qb, q[..., 0], many, many, 0.125) is None  # more chunks than a call takes
 
 
+@pytest.mark.parametrize("b,sq,sk,d,P", [
+    (1, 1, 1, 4, 1), (3, 33, 31, 32, 16), (2, 197, 70, 20, 5), (300, 100, 40, 32, 2), (513, 33, 33, 24, 2),  # 32, 64 and 128 rows a workgroup
+    (2, 65, 129, 64, 3), (300, 70, 33, 40, 1), (512, 129, 20, 64, 1),
+    (4, 171, 95, 80, 3), (280, 66, 32, 96, 2), (600, 32, 17, 88, 1),
+    (2, 40, 64, 128, 4), (260, 96, 50, 100, 1), (512, 64, 34, 128, 1),
+])
+def test_fp32_ring_in_one_launch_each_way(b, sq, sk, d, P, dev):
+    """fp32 rings over resident chunks against fp64: every kernel width with and without columns past the head size, every
+    number of rows a workgroup takes, groups of wavefronts without a step, lengths that end inside a step."""
+    torch.manual_seed(8)
+    scale = d**-0.5
+    q, dout = torch.randn(b, 1, sq, d), torch.randn(b, 1, sq, d)
+    ks, vs = ([torch.randn(b, 1, sk, d) for _ in range(P)] for _ in range(2))
+    want_o, want_l = oa.ring_forward(q.double(), [t.double() for t in ks], [t.double() for t in vs], scale)
+    on = lambda ts: [t.to(dev) for t in ts]  # noqa: E731
+    res = ja._resident_forward(q.to(dev), on(ks), on(vs), scale)
+    assert res is not None
+    out, lse = res
+    assert out.dtype == lse.dtype == torch.float32 and rel_l2(out, want_o) < 1e-5 and rel_l2(lse, want_l) < 1e-5
+    dq, dks, dvs = ja.ring_backward(dout.to(dev), q.to(dev), want_o.float().to(dev), want_l.float().to(dev), on(ks), on(vs), scale)
+    total = torch.zeros_like(q, dtype=torch.float64)
+    for k, v, dk, dv in zip(ks, vs, dks, dvs):
+        a, b_, c = oa.core_backward(dout.double(), q.double(), k.double(), v.double(), want_o, want_l, scale)
+        total += a
+        # with one key to attend the true dK is 0: what is left are roundings of the products that cancel
+        floor = 1e-6 * float((dout.double().unsqueeze(-2) * v.double().mean(-2, keepdim=True).unsqueeze(-2)).norm())
+        assert rel_l2(dv, c) < 1e-5 and float((dk.cpu().double() - b_).norm()) < 1e-5 * float(b_.norm()) + floor
+    assert float((dq.cpu().double() - total).norm()) < 1e-5 * float(total.norm()) + floor
+
+
 @pytest.mark.parametrize("d,n,nk", [(64, 192, 160), (32, 100, 70), (128, 64, 96)])
 def test_fp32_ring_step_takes_the_fused_merge(d, n, nk, dev):
     """``attend_step_`` on fp32 tensors at the head sizes of the fp32 matrix-core kernel: one launch that merges in
