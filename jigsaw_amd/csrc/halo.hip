@@ -263,7 +263,9 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs a, const T* __restri
 // One thread takes both ends of ROWS rows, 256 rows apart, all loads before the first store: the
 // two lines of a row are asked for together (neighbouring lanes: neighbouring rows, so whole
 // DRAM pages are read in one go instead of half now and half when the other face is packed),
-// and a lane has up to 2 * ROWS * ext loads in flight.
+// and a lane has up to 2 * ROWS * ext loads in flight. Non-temporal loads: of a line that a row gives one cell from, they
+// fetch half and leave none of it in the caches. 2^20 rows of 256 bytes 105 -> 42 us, 2^19 rows of 2048 bytes 57 -> 26
+// (whole lines fetched as 16-byte pieces by neighbouring lanes instead: 107 and 64).
 template <typename T>
 __global__ __launch_bounds__(256) void pack_w_faces_kernel(T* __restrict__ dlo, T* __restrict__ dhi,
                                                            const T* __restrict__ src, Box blo, Box bhi,
@@ -282,8 +284,8 @@ __global__ __launch_bounds__(256) void pack_w_faces_kernel(T* __restrict__ dlo, 
       const T* row = src + (((size_t)pl * Sd + (blo.org[0] + cd)) * Sh + (blo.org[1] + ch)) * (size_t)Sw;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        if (j < nlo) vlo[k][j] = row[blo.org[2] + j];
-        if (j < nhi) vhi[k][j] = row[bhi.org[2] + j];
+        if (j < nlo) vlo[k][j] = __builtin_nontemporal_load(row + blo.org[2] + j);
+        if (j < nhi) vhi[k][j] = __builtin_nontemporal_load(row + bhi.org[2] + j);
       }
     }
   }
@@ -482,7 +484,7 @@ struct RowPlan {
 typedef uint32_t u32x4_s4 __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int ROW_BATCH = 4;  // vectors a lane keeps in flight
 
-template <typename T>
+template <typename T, bool STREAM>
 __global__ __launch_bounds__(256) void assemble_rows_kernel(Table tab, T* __restrict__ dst,
                                                             Geom g, RowPlan pl) {
   constexpr int V = Bits<T>::V;
@@ -530,7 +532,10 @@ __global__ __launch_bounds__(256) void assemble_rows_kernel(Table tab, T* __rest
     for (int u = 0; u < ROW_BATCH; ++u) {
       const int j = lir + ((it0 + u) << pl.lpr_log2);
       val[u] = u32x4{0u, 0u, 0u, 0u};
-      if (j < n_full && s1 != nullptr) val[u] = *reinterpret_cast<const u32x4_any*>(s1 + j * V);
+      if (j < n_full && s1 != nullptr) {
+        const u32x4_any* const at = reinterpret_cast<const u32x4_any*>(s1 + j * V);
+        val[u] = STREAM ? __builtin_nontemporal_load(at) : *at;
+      }
     }
 #pragma unroll
     for (int u = 0; u < ROW_BATCH; ++u) {
@@ -1238,10 +1243,17 @@ extern "C" int jg_halo_assemble_3d(void* x_aug, const void* const src[27],
   const int V = 16 / elem_size;
   if (make_plan((unsigned long long)g.planes * Da * Ha, (Wa + V - 1) / V, Ha, Da, &pl)) {
     const unsigned blocks = (unsigned)((((unsigned long long)pl.nrows << pl.lpr_log2) + 255) / 256);
-    if (elem_size == 2)
-      assemble_rows_kernel<uint16_t><<<blocks, 256, 0, s>>>(tab, static_cast<uint16_t*>(x_aug), g, pl);
-    else
-      assemble_rows_kernel<uint32_t><<<blocks, 256, 0, s>>>(tab, static_cast<uint32_t*>(x_aug), g, pl);
+    // Rows of whole 128-byte lines: every line is fetched once, so non-temporally (nothing reads the tile again): the step of
+    // 2 x 32 -> 32 of 128^3 1069 -> 1054 us, at stride 2 of 4 x 64 -> 128 of 256 x 256 141 -> 138. A line that two rows share
+    // would be fetched twice (7 x 107 -> 75 of 644 x 348: 1400 -> 1416).
+    const bool stream_by = (long long)g.n[2] * elem_size % 128 == 0 && (reinterpret_cast<uintptr_t>(src[13]) & 127) == 0;
+    if (elem_size == 2) {
+      if (stream_by) assemble_rows_kernel<uint16_t, true><<<blocks, 256, 0, s>>>(tab, static_cast<uint16_t*>(x_aug), g, pl);
+      else assemble_rows_kernel<uint16_t, false><<<blocks, 256, 0, s>>>(tab, static_cast<uint16_t*>(x_aug), g, pl);
+    } else {
+      if (stream_by) assemble_rows_kernel<uint32_t, true><<<blocks, 256, 0, s>>>(tab, static_cast<uint32_t*>(x_aug), g, pl);
+      else assemble_rows_kernel<uint32_t, false><<<blocks, 256, 0, s>>>(tab, static_cast<uint32_t*>(x_aug), g, pl);
+    }
     JG_CHECK_LAUNCH("jg_halo_assemble_3d");
     return JG_OK;
   }
