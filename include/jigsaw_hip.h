@@ -453,6 +453,38 @@ int jg_proj_tn(void* gw, void* gb, const void* g, const void* x, int dtype, int 
                int64_t rows, int n, int c, int g_heads, int x_heads, int B, int H, int S, int D,
                void* workspace, size_t workspace_bytes, void* stream);
 
+/* Sums of partial results left for later. The _later variants of jg_proj_tn, jg_ln_plain_bwd_add / jg_ln_plain_bwd and
+ * jg_attn_swin_shifted_bwd write their partials, add what is to be summed to `later` (at most JG_MOST_REDUCTIONS; start
+ * with n = 0) and leave out the launches that sum: jg_reduce_many does all of the list in one launch on a stream ordered behind
+ * them, with the bits of those launches. Until then workspaces and outputs stay where they are. Where a variant
+ * has no partials (jg_proj_tn beyond its matrix kernels) or cannot leave its sums (outputs other than fp32) it sums by itself. */
+#define JG_MOST_REDUCTIONS 16
+typedef struct jg_reduction {
+  int32_t kind;   /* the library's own */
+  int32_t parts;
+  int64_t count;
+  const float* part;
+  float* out;
+  float* out2;
+} jg_reduction;
+typedef struct jg_reductions {
+  int32_t n;
+  jg_reduction job[JG_MOST_REDUCTIONS];
+} jg_reductions;
+int jg_reduce_many(const jg_reductions* all, void* stream);
+int jg_proj_tn_later(jg_reductions* later, void* gw, void* gb, const void* g, const void* x, int dtype, int grad_dtype,
+                     int64_t rows, int n, int c, int g_heads, int x_heads, int B, int H, int S, int D,
+                     void* workspace, size_t workspace_bytes, void* stream);
+/* add: NULL as jg_ln_plain_bwd */
+int jg_ln_plain_bwd_later(jg_reductions* later, void* gx, float* gw, float* gb, const void* g, const void* x,
+                          const float* mean, const float* rstd, const float* w, int64_t rows, int64_t cols, int g_dtype,
+                          int x_dtype, void* workspace, size_t workspace_bytes, const void* add, void* stream);
+int jg_attn_swin_shifted_bwd_later(jg_reductions* later, void* dq, void* dk, void* dv, float* dtable, const void* dout,
+                                   const void* q, const void* k, const void* v, const void* out, const float* lse,
+                                   const float* table, const uint8_t* side, int64_t images, int64_t heads, int64_t gh,
+                                   int64_t gw, int64_t shift_y, int64_t shift_x, int64_t d, float scale, int dtype,
+                                   void* workspace, size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------- *
  * Online-softmax / log-sum-exp merge of ring attention (HBM-bound)
  * ------------------------------------------------------------------------- */

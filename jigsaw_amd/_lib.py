@@ -312,6 +312,23 @@ SIGNATURES: dict[str, tuple] = {
          c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_float, c_int, c_void_p, c_size_t,
          c_void_p],
     ),
+    "jg_attn_swin_shifted_bwd_later": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+         c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_float, c_int, c_void_p, c_size_t,
+         c_void_p],
+    ),
+    "jg_proj_tn_later": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
+         c_int, c_void_p, c_size_t, c_void_p],
+    ),
+    "jg_ln_plain_bwd_later": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int,
+         c_int, c_void_p, c_size_t, c_void_p, c_void_p],
+    ),
+    "jg_reduce_many": (c_int, [c_void_p, c_void_p]),
     "jg_attn_swin_bwd_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64, c_int64]),
     "jg_attn_swin_bwd": (
         c_int,

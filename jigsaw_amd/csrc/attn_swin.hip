@@ -26,6 +26,7 @@
 //              plain read, add, write per register is exact and its order fixed), writes the bins
 //              out, and two small kernels add the entries' bins per head in a fixed order.
 #include "attn_window_common.h"
+#include "reductions.h"
 
 namespace {
 
@@ -426,31 +427,11 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_swin_bwd_kernel(SwinArgs p
   }
 }
 
-// Table gradient, stage 1: block (head, chunk) adds the bins of its wavefronts, one after the other;
-// thread i < 450 owns bin i. stage 2: block `head` adds the chunks and the two lane halves.
-constexpr int CHUNKS = 32;
-__global__ __launch_bounds__(512) void swin_bins_stage1(const float* __restrict__ bins, float* __restrict__ part,
-                                                        long long workers, int heads) {
-  const int head = blockIdx.x, chunk = blockIdx.y, i = threadIdx.x;
-  if (i >= BINS) return;
-  const long long groups = workers / heads;  // wavefronts of one head
-  const long long per = (groups + CHUNKS - 1) / CHUNKS;
-  long long g0 = chunk * per, g1 = g0 + per;
-  if (g1 > groups) g1 = groups;
-  float acc = 0.0f;
-#pragma unroll 8
-  for (long long g = g0; g < g1; ++g) acc += bins[(g * heads + head) * BINS + i];
-  part[((size_t)head * CHUNKS + chunk) * BINS + i] = acc;
-}
-__global__ __launch_bounds__(256) void swin_bins_stage2(const float* __restrict__ part, float* __restrict__ dtable, int heads) {
-  const int head = blockIdx.x, i = threadIdx.x;
-  if (i >= ROWS) return;
-  float acc = 0.0f;
-  for (int c = 0; c < CHUNKS; ++c) {
-    const float* pc = part + ((size_t)head * CHUNKS + c) * BINS;
-    acc += pc[i] + pc[ROWS + i];
-  }
-  dtable[(size_t)i * heads + head] = acc;
+// Table gradient from the wavefronts' bins.
+static_assert(ROWS == jg::RED_BINS && BINS == 2 * jg::RED_BINS, "the layout of the bins");
+__global__ __launch_bounds__(jg::RED_THREADS) void swin_bins_kernel(const float* __restrict__ bins, float* __restrict__ dtable, int workers, int heads) {
+  __shared__ float sm[2][32][33];
+  jg::reduce_table(sm, bins, dtable, workers, heads, blockIdx.x);
 }
 
 int check(const char* who, int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t shift_y, int64_t shift_x, int64_t d,
@@ -517,20 +498,18 @@ extern "C" int jg_attn_swin_shifted_fwd(void* out, float* lse, const void* q, co
   return JG_OK;
 }
 
-// Workspace of jg_attn_swin_bwd when the table gradient is wanted: the bins of every entry and
-// the chunk sums of the first reduction stage.
+// Workspace of jg_attn_swin_bwd when the table gradient is wanted: the bins of its wavefronts, at most one an entry.
 extern "C" size_t jg_attn_swin_bwd_workspace_bytes(int64_t images, int64_t heads, int64_t gh, int64_t gw) {
   if (images <= 0 || heads <= 0 || gh <= 0 || gw <= 0) return 0;
   const size_t entries = (size_t)images * (size_t)((gh / WIN) * (gw / WIN)) * (size_t)heads;
-  return (entries + (size_t)heads * CHUNKS) * BINS * sizeof(float);
+  return entries * BINS * sizeof(float);
 }
 
-extern "C" int jg_attn_swin_shifted_bwd(void* dq, void* dk, void* dv, float* dtable, const void* dout, const void* q,
-                                        const void* k, const void* v, const void* out, const float* lse,
-                                        const float* table, const uint8_t* side, int64_t images, int64_t heads, int64_t gh,
-                                        int64_t gw, int64_t shift_y, int64_t shift_x, int64_t d, float scale, int dtype,
-                                        void* workspace, size_t workspace_bytes, void* stream) {
-  const char* who = "jg_attn_swin_bwd";
+// later: NULL, or where the sum of the bins is left
+static int swin_bwd(const char* who, jg_reductions* later, void* dq, void* dk, void* dv, float* dtable, const void* dout, const void* q,
+                    const void* k, const void* v, const void* out, const float* lse, const float* table, const uint8_t* side, int64_t images,
+                    int64_t heads, int64_t gh, int64_t gw, int64_t shift_y, int64_t shift_x, int64_t d, float scale, int dtype, void* workspace,
+                    size_t workspace_bytes, void* stream) {
   int rc = check(who, images, heads, gh, gw, shift_y, shift_x, d, dtype, scale);
   if (rc) return rc;
   JG_REQUIRE(dq && dk && dv && dout && q && k && v && out && lse && table, "%s: NULL pointer", who);
@@ -567,16 +546,34 @@ extern "C" int jg_attn_swin_shifted_bwd(void* dq, void* dk, void* dv, float* dta
   if (dtable != nullptr) {
     attn_swin_bwd_kernel<true><<<grid, WAVES * 64, BWD_LDS, s>>>(a);
     JG_CHECK_LAUNCH(who);
-    float* part = a.bins + (size_t)workers * BINS;
-    swin_bins_stage1<<<dim3((unsigned)heads, CHUNKS), 512, 0, s>>>(a.bins, part, workers, (int)heads);
-    JG_CHECK_LAUNCH(who);
-    swin_bins_stage2<<<dim3((unsigned)heads), 256, 0, s>>>(part, dtable, (int)heads);
+    if (later != nullptr) return jg::add_reduction(later, jg::RED_TABLE, (int)workers, heads, a.bins, dtable, nullptr);
+    swin_bins_kernel<<<(unsigned)heads * jg::RED_TABLE_BLOCKS, jg::RED_THREADS, 0, s>>>(a.bins, dtable, (int)workers, (int)heads);
     JG_CHECK_LAUNCH(who);
   } else {
     attn_swin_bwd_kernel<false><<<grid, WAVES * 64, BWD_LDS, s>>>(a);
     JG_CHECK_LAUNCH(who);
   }
   return JG_OK;
+}
+
+extern "C" int jg_attn_swin_shifted_bwd(void* dq, void* dk, void* dv, float* dtable, const void* dout, const void* q,
+                                        const void* k, const void* v, const void* out, const float* lse,
+                                        const float* table, const uint8_t* side, int64_t images, int64_t heads, int64_t gh,
+                                        int64_t gw, int64_t shift_y, int64_t shift_x, int64_t d, float scale, int dtype,
+                                        void* workspace, size_t workspace_bytes, void* stream) {
+  return swin_bwd("jg_attn_swin_bwd", nullptr, dq, dk, dv, dtable, dout, q, k, v, out, lse, table, side, images, heads, gh, gw, shift_y, shift_x, d,
+                  scale, dtype, workspace, workspace_bytes, stream);
+}
+
+extern "C" int jg_attn_swin_shifted_bwd_later(jg_reductions* later, void* dq, void* dk, void* dv, float* dtable, const void* dout, const void* q,
+                                              const void* k, const void* v, const void* out, const float* lse, const float* table,
+                                              const uint8_t* side, int64_t images, int64_t heads, int64_t gh, int64_t gw, int64_t shift_y,
+                                              int64_t shift_x, int64_t d, float scale, int dtype, void* workspace, size_t workspace_bytes,
+                                              void* stream) {
+  const char* who = "jg_attn_swin_bwd_later";
+  JG_REQUIRE(later != nullptr, "%s: NULL pointer", who);
+  return swin_bwd(who, later, dq, dk, dv, dtable, dout, q, k, v, out, lse, table, side, images, heads, gh, gw, shift_y, shift_x, d, scale, dtype, workspace,
+                  workspace_bytes, stream);
 }
 
 extern "C" int jg_attn_swin_fwd(void* out, float* lse, const void* q, const void* k, const void* v, const float* table,

@@ -472,12 +472,24 @@ void nt_fused(const at::Tensor& out, const at::Tensor& aux, int epilogue, const 
         "jg_proj_nt_fused");
 }
 // (gw, gb): gradients of a weight (n, c) and its bias from the gradient and the input of its layer
+// With `later` the sums of the partials are left to it, and the partials to `held`.
+struct Later {
+  jg_reductions sums = {};
+  List held;
+};
 std::pair<at::Tensor, at::Tensor> tn(const at::Tensor& g, const at::Tensor& x, int64_t rows, int64_t n, int64_t c, bool g_heads, bool x_heads, const Heads& l,
-                                     bool need_b, at::ScalarType grad_type, void* s) {
+                                     bool need_b, at::ScalarType grad_type, void* s, Later* later = nullptr) {
   const auto options = g.options().dtype(grad_type);
   const at::Tensor gw = at::empty({n, c}, options), gb = need_b ? at::empty({n}, options) : at::Tensor();
   const size_t nbytes = jg_proj_tn_workspace(rows, n, c);
   const at::Tensor ws = bytes(g, std::max<size_t>(nbytes, 16));
+  if (later != nullptr) {
+    later->held.push_back(ws);
+    check(jg_proj_tn_later(&later->sums, gw.data_ptr(), need_b ? gb.data_ptr() : nullptr, g.data_ptr(), x.data_ptr(), code_of(g),
+                           grad_type == at::kFloat ? JG_F32 : code_of(g), rows, n, c, g_heads, x_heads, l.b, l.h, l.s, l.d, ws.data_ptr(), nbytes, s),
+          "jg_proj_tn_later");
+    return {gw, gb};
+  }
   check(jg_proj_tn(gw.data_ptr(), need_b ? gb.data_ptr() : nullptr, g.data_ptr(), x.data_ptr(), code_of(g), grad_type == at::kFloat ? JG_F32 : code_of(g),
                    rows, n, c, g_heads, x_heads, l.b, l.h, l.s, l.d, ws.data_ptr(), nbytes, s),
         "jg_proj_tn");
@@ -598,16 +610,17 @@ class SwinPass {
     const int64_t c = x.size(3), rows = l.b * l.s, hidden = pre.size(3);
     const Heads flat;
     at::Tensor g[PARAMS];
-    std::tie(g[FC2_W], g[FC2_B]) = tn(grad, act, rows, c, hidden, false, false, flat, true, at::kFloat, s);
+    Later later;  // every parameter's sums of partials in one launch at the end
+    std::tie(g[FC2_W], g[FC2_B]) = tn(grad, act, rows, c, hidden, false, false, flat, true, at::kFloat, s, &later);
     const at::Tensor dpre = at::empty_like(pre);
     nt_fused(dpre, pre, JG_EPI_DGELU, grad, wt[3], nullptr, rows, s);
-    std::tie(g[FC1_W], g[FC1_B]) = tn(dpre, y2, rows, hidden, c, false, false, flat, true, at::kFloat, s);
+    std::tie(g[FC1_W], g[FC1_B]) = tn(dpre, y2, rows, hidden, c, false, false, flat, true, at::kFloat, s, &later);
     const at::Tensor gy2 = at::empty_like(x);
     nt(gy2, dpre, wt[2], nullptr, rows, false, false, flat, s);
-    const at::Tensor gx1 = norm_backward(gy2, grad, x1, mean2, rstd2, n2w, true, &g[N2W], &g[N2B], s);
+    const at::Tensor gx1 = norm_backward(gy2, grad, x1, mean2, rstd2, n2w, true, &g[N2W], &g[N2B], later, s);
     const at::Tensor gout = at::empty_like(out);
     nt(gout, gx1, wt[1], nullptr, rows, false, true, l, s);
-    std::tie(g[PROJ_W], g[PROJ_B]) = tn(gx1, out, rows, c, c, false, true, l, true, at::kFloat, s);
+    std::tie(g[PROJ_W], g[PROJ_B]) = tn(gx1, out, rows, c, c, false, true, l, true, at::kFloat, s, &later);
     const at::Tensor dqkv = at::empty_like(qkv);
     g[TABLE] = at::empty_like(table);
     const size_t nbytes = jg_attn_swin_bwd_workspace_bytes(l.b, l.h, h, w);
@@ -615,14 +628,15 @@ class SwinPass {
     const char* const q = static_cast<const char*>(qkv.data_ptr());
     char* const dq = static_cast<char*>(dqkv.data_ptr());
     const int64_t part = 2 * rows * c;
-    check(jg_attn_swin_shifted_bwd(dq, dq + part, dq + 2 * part, g[TABLE].data_ptr<float>(), gout.data_ptr(), q, q + part, q + 2 * part, out.data_ptr(),
-                                   lse.data_ptr<float>(), table.data_ptr<float>(), codes(), l.b, l.h, h, w, shift_y(), shift_x(), 32, (float)scale(), JG_BF16,
-                                   ws.data_ptr(), nbytes, s),
-          "jg_attn_swin_shifted_bwd");
+    check(jg_attn_swin_shifted_bwd_later(&later.sums, dq, dq + part, dq + 2 * part, g[TABLE].data_ptr<float>(), gout.data_ptr(), q, q + part, q + 2 * part,
+                                         out.data_ptr(), lse.data_ptr<float>(), table.data_ptr<float>(), codes(), l.b, l.h, h, w, shift_y(), shift_x(), 32,
+                                         (float)scale(), JG_BF16, ws.data_ptr(), nbytes, s),
+          "jg_attn_swin_shifted_bwd_later");
     const at::Tensor gy = at::empty_like(x);
     nt(gy, dqkv, wt[0], nullptr, rows, true, false, l, s);
-    std::tie(g[QKV_W], g[QKV_B]) = tn(dqkv, y1, rows, 3 * c, c, true, false, l, true, at::kFloat, s);
-    const at::Tensor gx = norm_backward(gy, gx1, x, mean1, rstd1, n1w, need_x, &g[N1W], &g[N1B], s);
+    std::tie(g[QKV_W], g[QKV_B]) = tn(dqkv, y1, rows, 3 * c, c, true, false, l, true, at::kFloat, s, &later);
+    const at::Tensor gx = norm_backward(gy, gx1, x, mean1, rstd1, n1w, need_x, &g[N1W], &g[N1B], later, s);
+    check(jg_reduce_many(&later.sums, s), "jg_reduce_many");
     py::tuple all(1 + PARAMS);
     all[0] = need_x ? py::cast(gx) : py::none();
     for (int i = 0; i < PARAMS; ++i) all[1 + i] = py::cast(g[i]);
@@ -664,21 +678,18 @@ class SwinPass {
   }
   // the gradient of the norm's input with what reaches it past the norm (`over`) added, if wanted; gw, gb
   static at::Tensor norm_backward(const at::Tensor& g, const at::Tensor& over, const at::Tensor& x, const at::Tensor& mean, const at::Tensor& rstd,
-                                  const at::Tensor& w, bool need_x, at::Tensor* gw, at::Tensor* gb, void* s) {
+                                  const at::Tensor& w, bool need_x, at::Tensor* gw, at::Tensor* gb, Later& later, void* s) {
     const int64_t cols = x.size(-1), rows = x.numel() / cols;
     const at::Tensor gx = need_x ? at::empty_like(x) : at::Tensor();
     *gw = f32(x, {cols});
     *gb = f32(x, {cols});
     const size_t nbytes = jg_ln_plain_bwd_workspace_bytes(rows, cols);
     const at::Tensor ws = bytes(x, std::max<size_t>(nbytes, 4));
-    if (need_x)
-      check(jg_ln_plain_bwd_add(gx.data_ptr(), gw->data_ptr<float>(), gb->data_ptr<float>(), g.data_ptr(), x.data_ptr(), mean.data_ptr<float>(),
-                                rstd.data_ptr<float>(), w.data_ptr<float>(), rows, cols, JG_BF16, JG_BF16, ws.data_ptr(), nbytes, over.data_ptr(), s),
-            "jg_ln_plain_bwd_add");
-    else
-      check(jg_ln_plain_bwd(nullptr, gw->data_ptr<float>(), gb->data_ptr<float>(), g.data_ptr(), x.data_ptr(), mean.data_ptr<float>(),
-                            rstd.data_ptr<float>(), w.data_ptr<float>(), rows, cols, JG_BF16, JG_BF16, ws.data_ptr(), nbytes, s),
-            "jg_ln_plain_bwd");
+    later.held.push_back(ws);
+    check(jg_ln_plain_bwd_later(&later.sums, need_x ? gx.data_ptr() : nullptr, gw->data_ptr<float>(), gb->data_ptr<float>(), g.data_ptr(), x.data_ptr(),
+                                mean.data_ptr<float>(), rstd.data_ptr<float>(), w.data_ptr<float>(), rows, cols, JG_BF16, JG_BF16, ws.data_ptr(), nbytes,
+                                need_x ? over.data_ptr() : nullptr, s),
+          "jg_ln_plain_bwd_later");
     return gx;
   }
   const uint8_t* codes() const { return side.defined() ? side.data_ptr<uint8_t>() : nullptr; }

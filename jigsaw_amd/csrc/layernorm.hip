@@ -7,7 +7,7 @@
 // Reference behaviour restated here:
 //   jigsaw/modules/normalization/_functional.py:45-58   (forward)
 //   jigsaw/modules/normalization/_functional.py:141-175 (backward)
-#include "jg_common.h"
+#include "reductions.h"
 
 #include <mutex>
 #include <type_traits>
@@ -250,12 +250,8 @@ __global__ __launch_bounds__(kThreads) void ln_partial_bwd_kernel(
   }
 }
 
-// Stage 2: a block owns 16 consecutive columns, so that a wavefront reads 64 bytes of 4 block partials at a time; its 16
-// wavefronts take the partials k = 4 w + lane / 16, ... + 64, ... in 4 independent chains each, and all chain sums are
-// added in a fixed order (deterministic). Bound by the latency of a chain: 1024 partials of
-// 128 columns 7.2 us with 64 columns a block (two blocks), 4.9 us with 16.
-constexpr int kReduceWaves = 16, kReduceCols = 16;
-static_assert(kReduceWaves * 64 == 4 * kReduceWaves * kReduceCols, "4 partials a wavefront");
+// Stage 2: jg::reduce_columns
+constexpr int kReduceWaves = jg::RED_WAVES, kReduceCols = jg::RED_COLS;
 __device__ __forceinline__ void store_as(void* p, long long i, float v, int dtype) {
   if (dtype == JG_F32) static_cast<float*>(p)[i] = v;
   else if (dtype == JG_BF16) static_cast<uint16_t*>(p)[i] = Elem<JG_BF16>::down(v);
@@ -265,44 +261,10 @@ __global__ __launch_bounds__(kReduceWaves * 64) void ln_colreduce_kernel(void* _
                                                                          const float* __restrict__ part,
                                                                          int nblocks, long long cols) {
   __shared__ float red[2][kReduceWaves][kReduceCols];
-  const int col = threadIdx.x % kReduceCols, first = threadIdx.x / kReduceCols;
-  constexpr int STEP = 4 * kReduceWaves;  // partials the block reads at a time
-  const long long c = (long long)blockIdx.x * kReduceCols + col;
-  float a[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f};
-  if (c < cols) {
-    int k = first;
-    for (; k + 3 * STEP < nblocks; k += 4 * STEP) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        a[u] += part[((long long)(k + STEP * u) * 2 + 0) * cols + c];
-        b[u] += part[((long long)(k + STEP * u) * 2 + 1) * cols + c];
-      }
-    }
-    for (; k < nblocks; k += STEP) {
-      a[0] += part[((long long)k * 2 + 0) * cols + c];
-      b[0] += part[((long long)k * 2 + 1) * cols + c];
-    }
-  }
-  float sw = (a[0] + a[1]) + (a[2] + a[3]), sb = (b[0] + b[1]) + (b[2] + b[3]);
-#pragma unroll
-  for (int o = kReduceCols; o < kWave; o <<= 1) {
-    sw += __shfl_xor(sw, o, kWave);
-    sb += __shfl_xor(sb, o, kWave);
-  }
-  if (first % 4 == 0) {
-    red[0][first / 4][col] = sw;
-    red[1][first / 4][col] = sb;
-  }
-  __syncthreads();
-  if (first != 0 || c >= cols) return;
-  sw = sb = 0.0f;
-#pragma unroll
-  for (int i = 0; i < kReduceWaves; ++i) {
-    sw += red[0][i][col];
-    sb += red[1][i][col];
-  }
-  if (gw != nullptr) store_as(gw, c, sw, dtype);
-  if (gb != nullptr) store_as(gb, c, sb, dtype);
+  jg::reduce_columns(red, part, nblocks, cols, blockIdx.x, [=](long long c, float sw, float sb) {
+    if (gw != nullptr) store_as(gw, c, sw, dtype);
+    if (gb != nullptr) store_as(gb, c, sb, dtype);
+  });
 }
 
 template <int DT>
@@ -1403,7 +1365,7 @@ extern "C" size_t jg_ln_plain_bwd_workspace_bytes(int64_t rows, int64_t cols) {
 static int plain_bwd_common(const char* who, void* gx, float* gw, float* gb, const void* g, const void* x,
                             const float* mean, const float* rstd, const float* w, int64_t rows, int64_t cols,
                             int g_dtype, int x_dtype, void* workspace, size_t workspace_bytes, const void* add,
-                            void* stream) {
+                            jg_reductions* later, void* stream) {
   JG_REQUIRE(g && x && mean && rstd && w, "%s: NULL pointer", who);
   JG_REQUIRE(add == nullptr || (gx != nullptr && aligned16(add)), "%s: add needs gx and 16-byte alignment", who);
   JG_REQUIRE(rows >= 0 && cols >= 1, "%s: bad shape (%lld, %lld)", who, (long long)rows, (long long)cols);
@@ -1445,6 +1407,7 @@ static int plain_bwd_common(const char* who, void* gx, float* gw, float* gb, con
   }
 #undef JG_GO
   JG_CHECK_LAUNCH(who);
+  if (want_cols && later != nullptr) return jg::add_reduction(later, jg::RED_COLUMNS, plain_blocks(rows, cols), cols, part, gw, gb);
   if (want_cols) {
     ln_colreduce_kernel<<<(unsigned)((cols + kReduceCols - 1) / kReduceCols), kReduceWaves * 64, 0, s>>>(gw, gb, JG_F32, part, plain_blocks(rows, cols), cols);
     JG_CHECK_LAUNCH(who);
@@ -1457,7 +1420,7 @@ extern "C" int jg_ln_plain_bwd(void* gx, float* gw, float* gb, const void* g, co
                                int64_t cols, int g_dtype, int x_dtype, void* workspace,
                                size_t workspace_bytes, void* stream) {
   return plain_bwd_common("jg_ln_plain_bwd", gx, gw, gb, g, x, mean, rstd, w, rows, cols, g_dtype, x_dtype, workspace,
-                          workspace_bytes, nullptr, stream);
+                          workspace_bytes, nullptr, nullptr, stream);
 }
 
 extern "C" int jg_ln_plain_bwd_add(void* gx, float* gw, float* gb, const void* g, const void* x,
@@ -1467,5 +1430,15 @@ extern "C" int jg_ln_plain_bwd_add(void* gx, float* gw, float* gb, const void* g
   const char* who = "jg_ln_plain_bwd_add";
   JG_REQUIRE(add != nullptr && gx != nullptr, "%s: NULL pointer", who);
   return plain_bwd_common(who, gx, gw, gb, g, x, mean, rstd, w, rows, cols, g_dtype, x_dtype, workspace,
-                          workspace_bytes, add, stream);
+                          workspace_bytes, add, nullptr, stream);
+}
+
+extern "C" int jg_ln_plain_bwd_later(jg_reductions* later, void* gx, float* gw, float* gb, const void* g, const void* x,
+                                     const float* mean, const float* rstd, const float* w, int64_t rows, int64_t cols,
+                                     int g_dtype, int x_dtype, void* workspace, size_t workspace_bytes, const void* add,
+                                     void* stream) {
+  const char* who = "jg_ln_plain_bwd_later";
+  JG_REQUIRE(later != nullptr, "%s: NULL pointer", who);
+  return plain_bwd_common(who, gx, gw, gb, g, x, mean, rstd, w, rows, cols, g_dtype, x_dtype, workspace, workspace_bytes, add,
+                          later, stream);
 }

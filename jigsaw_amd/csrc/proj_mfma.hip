@@ -24,7 +24,7 @@
 // proj_generic_kernel covers the other dtypes and unaligned shapes with plain FMAs.
 #include <type_traits>
 
-#include "jg_common.h"
+#include "reductions.h"
 
 namespace {
 
@@ -641,56 +641,32 @@ struct ReduceArgs {
 
 template <int W>
 __global__ __launch_bounds__(64 * W) void proj_reduce_kernel(ReduceArgs a) {
-  __shared__ f32x4 sm[W][64];
+  __shared__ float4 sm[W][64];
   const size_t blocks_w = (a.count_w + 255) / 256;
   const bool second = blockIdx.x >= blocks_w;
-  void* out_any = second ? a.out_b : a.out_w;
+  void* const out = second ? a.out_b : a.out_w;
   const float* part = second ? a.part_b : a.part_w;
   const size_t count = second ? a.count_b : a.count_w;
-  const int q = threadIdx.x & 63, grp = threadIdx.x >> 6;
-  const size_t i0 = (blockIdx.x - (second ? blocks_w : 0)) * 256 + (size_t)q * 4;
   // every split's slice starts 16-byte aligned when the count is a multiple of 4 and the base is aligned
-  const bool vec = (count & 3) == 0 && (reinterpret_cast<uintptr_t>(part) & 15) == 0 &&
-                   (reinterpret_cast<uintptr_t>(out_any) & 15) == 0;
-  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (i0 < count) {
-    if (vec) {
-      for (int k = grp; k < a.splits; k += W) acc += *reinterpret_cast<const f32x4*>(part + (size_t)k * count + i0);
-    } else {
-      for (int k = grp; k < a.splits; k += W)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (i0 + e < count) acc[e] += part[(size_t)k * count + i0 + e];
-    }
-  }
-  sm[grp][q] = acc;
-  __syncthreads();
-  if (grp != 0 || i0 >= count) return;
-  f32x4 t = sm[0][q];
-#pragma unroll
-  for (int w = 1; w < W; ++w) t += sm[w][q];
-  if (a.out32) {
-    float* o32 = static_cast<float*>(out_any);
-    if (vec) {
-      *reinterpret_cast<f32x4*>(o32 + i0) = t;
+  const bool vec = jg::slices_vec(part, out, count), out32 = a.out32 != 0;
+  jg::reduce_slices<W>(sm, part, count, a.splits, vec, blockIdx.x - (second ? blocks_w : 0), threadIdx.x >> 6, threadIdx.x & 63, [=](size_t i0, float4 t) {
+    const float v[4] = {t.x, t.y, t.z, t.w};
+    if (out32 && vec) {
+      *reinterpret_cast<float4*>(static_cast<float*>(out) + i0) = t;
+    } else if (vec) {
+      u32x2 o;
+      o.x = (uint32_t)jg::f32_to_bf16(v[0]) | ((uint32_t)jg::f32_to_bf16(v[1]) << 16);
+      o.y = (uint32_t)jg::f32_to_bf16(v[2]) | ((uint32_t)jg::f32_to_bf16(v[3]) << 16);
+      *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(out) + i0) = o;
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (i0 + e < count) o32[i0 + e] = t[e];
+        if (i0 + e < count) {
+          if (out32) static_cast<float*>(out)[i0 + e] = v[e];
+          else static_cast<uint16_t*>(out)[i0 + e] = jg::f32_to_bf16(v[e]);
+        }
     }
-    return;
-  }
-  uint16_t* out = static_cast<uint16_t*>(out_any);
-  if (vec) {
-    u32x2 o;
-    o.x = (uint32_t)jg::f32_to_bf16(t[0]) | ((uint32_t)jg::f32_to_bf16(t[1]) << 16);
-    o.y = (uint32_t)jg::f32_to_bf16(t[2]) | ((uint32_t)jg::f32_to_bf16(t[3]) << 16);
-    *reinterpret_cast<u32x2*>(out + i0) = o;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (i0 + e < count) out[i0 + e] = jg::f32_to_bf16(t[e]);
-  }
+  });
 }
 
 // ------------------------------------------------------------------- generic
@@ -1061,10 +1037,9 @@ size_t jg_proj_tn_workspace(int64_t rows, int n, int c) {
   return splits * ((size_t)n * c + n) * sizeof(float);
 }
 
-int jg_proj_tn(void* gw, void* gb, const void* g, const void* x, int dtype, int grad_dtype, int64_t rows, int n, int c,
-               int g_heads, int x_heads, int B, int H, int S, int D, void* workspace, size_t workspace_bytes,
-               void* stream) {
-  const char* who = "jg_proj_tn";
+// later: NULL, or where the sums of the splits are left
+static int proj_tn_common(const char* who, jg_reductions* later, void* gw, void* gb, const void* g, const void* x, int dtype, int grad_dtype, int64_t rows,
+                          int n, int c, int g_heads, int x_heads, int B, int H, int S, int D, void* workspace, size_t workspace_bytes, void* stream) {
   JG_REQUIRE(gw && g && x, "%s: null pointer", who);
   JG_REQUIRE(jg::dtype_size(dtype) != 0, "%s: unknown dtype %d", who, dtype);
   JG_REQUIRE(grad_dtype == dtype || grad_dtype == JG_F32, "%s: gradient dtype %d with operand dtype %d", who, grad_dtype,
@@ -1117,6 +1092,10 @@ int jg_proj_tn(void* gw, void* gb, const void* g, const void* x, int dtype, int 
   else
     rc = far ? launch_tn<2, 2, 2, 2, uint64_t>(p, splits, s, who) : launch_tn<2, 2, 2, 2, uint32_t>(p, splits, s, who);
   if (rc) return rc;
+  if (later != nullptr && out32) {
+    rc = jg::add_reduction(later, jg::RED_SLICES, splits, (int64_t)n * c, p.part, static_cast<float*>(gw), nullptr);
+    return rc != JG_OK || gb == nullptr ? rc : jg::add_reduction(later, jg::RED_SLICES, splits, n, p.bias_part, static_cast<float*>(gb), nullptr);
+  }
   ReduceArgs ra{};
   ra.out_w = gw;
   ra.part_w = p.part;
@@ -1127,10 +1106,23 @@ int jg_proj_tn(void* gw, void* gb, const void* g, const void* x, int dtype, int 
   ra.splits = splits;
   ra.out32 = out32 ? 1 : 0;
   const size_t blocks = (ra.count_w + 255) / 256 + (ra.count_b + 255) / 256;
-  if (splits >= 32) proj_reduce_kernel<16><<<(unsigned)blocks, 1024, 0, s>>>(ra);
+  if (jg::slice_waves(splits) == 16) proj_reduce_kernel<16><<<(unsigned)blocks, 1024, 0, s>>>(ra);
   else proj_reduce_kernel<4><<<(unsigned)blocks, 256, 0, s>>>(ra);
   JG_CHECK_LAUNCH(who);
   return JG_OK;
+}
+
+int jg_proj_tn(void* gw, void* gb, const void* g, const void* x, int dtype, int grad_dtype, int64_t rows, int n, int c,
+               int g_heads, int x_heads, int B, int H, int S, int D, void* workspace, size_t workspace_bytes,
+               void* stream) {
+  return proj_tn_common("jg_proj_tn", nullptr, gw, gb, g, x, dtype, grad_dtype, rows, n, c, g_heads, x_heads, B, H, S, D, workspace, workspace_bytes, stream);
+}
+
+int jg_proj_tn_later(jg_reductions* later, void* gw, void* gb, const void* g, const void* x, int dtype, int grad_dtype, int64_t rows, int n, int c,
+                     int g_heads, int x_heads, int B, int H, int S, int D, void* workspace, size_t workspace_bytes, void* stream) {
+  const char* who = "jg_proj_tn_later";
+  JG_REQUIRE(later != nullptr, "%s: null pointer", who);
+  return proj_tn_common(who, later, gw, gb, g, x, dtype, grad_dtype, rows, n, c, g_heads, x_heads, B, H, S, D, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

@@ -216,6 +216,13 @@ def test_native_block_has_the_bits_of_the_python_route(batch, n, dim, shift, dev
         assert torch.equal(a, want)
 
 
+@pytest.mark.parametrize("batch,n,dim,shift", [(2, (128, 128), 128, 4), (1, (256, 136), 96, 0)])
+def test_sums_left_for_one_launch_have_the_bits_of_their_own(batch, n, dim, shift, dev, monkeypatch):
+    """Sizes whose partials are many (32 splits and more, several workgroups of columns): the native backward sums them all in
+    one launch, the Python route each behind its kernel."""
+    test_native_block_has_the_bits_of_the_python_route(batch, n, dim, shift, dev, monkeypatch)
+
+
 @pytest.mark.parametrize("shift", [0, 4])
 def test_block_step_recorded_in_a_hip_graph_replays_the_eager_step(shift, dev):
     """``SwinBlock.captured_step``: forward + backward recorded once, replayed several times with eager
