@@ -507,9 +507,11 @@ __global__ __launch_bounds__(kThreads) void ln_plain_fwd_kernel(
 }
 
 // gx = rstd * (g w - mean_c(g w) - x_hat * mean_c(g w x_hat)); column partials of g x_hat and g
-// per block in part[blk][which][col] (ln_colreduce_kernel finishes them).
+// per block in part[blk][which][col] (ln_colreduce_kernel finishes them). Rows of one vector a lane (up to 512 columns) fit 128
+// registers and 16 KB of LDS, so that four workgroups a compute unit cover each other's memory latency where two
+// did (176 registers, 64 KB): with the residual added 20 to 23 -> 16 us at 65536 x 128, 46.5 -> 31.5 at 76608 x 256.
 template <int GDT, int XDT, int CH, int U>
-__global__ __launch_bounds__(kThreads) void ln_plain_bwd_kernel(
+__global__ __launch_bounds__(kThreads, CH == 1 ? 4 : 1) void ln_plain_bwd_kernel(
     typename Elem<XDT>::T* __restrict__ gx, float* __restrict__ part,
     const typename Elem<GDT>::T* __restrict__ g, const typename Elem<XDT>::T* __restrict__ x,
     const float* __restrict__ mean, const float* __restrict__ rstd, const float* __restrict__ w,
@@ -611,7 +613,7 @@ __global__ __launch_bounds__(kThreads) void ln_plain_bwd_kernel(
         agw[k][i] += __shfl_xor(agw[k][i], o, kWave);
         agb[k][i] += __shfl_xor(agb[k][i], o, kWave);
       }
-  __shared__ float red[kWavesPerBlock][2][kPlainChunks * kWave * kPlainVec];
+  __shared__ float red[kWavesPerBlock][2][CH * kWave * kPlainVec];
   if (sub == 0) {
 #pragma unroll
     for (int k = 0; k < CH; ++k)
