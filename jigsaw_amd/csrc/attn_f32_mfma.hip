@@ -230,12 +230,13 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_fwd_kernel(jg::ChunkTa
 #pragma unroll
     for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m, mx);  // finite: key 0 of every step exists
-    const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+    const float m_new = fmaxf(m, mx);
+    const float ms = m_new == -INFINITY ? 0.0f : m_new;  // steps whose scores are all -inf (infinite keys) weigh nothing
+    const float alpha = __builtin_amdgcn_exp2f(m - ms);
     float sum = 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      s[i] = __builtin_amdgcn_exp2f(s[i] - m_new);
+      s[i] = __builtin_amdgcn_exp2f(s[i] - ms);
       sum += s[i];
     }
     sum += __shfl_xor(sum, 32, 64);
@@ -271,8 +272,8 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_fwd_kernel(jg::ChunkTa
       const float* at = smem + ((k - 1) * R + me.row_wave) * PART + me.lane;
       const float mk = at[NT * 16 * 64], lk = at[(NT * 16 + 1) * 64];
       if (per_chunk * p.chunks <= k) break;  // a group that had no step
-      const float top = fmaxf(m, mk);
-      const float mine = __builtin_amdgcn_exp2f(m - top), other = __builtin_amdgcn_exp2f(mk - top);
+      const float top = fmaxf(m, mk), ts = top == -INFINITY ? 0.0f : top;
+      const float mine = __builtin_amdgcn_exp2f(m - ts), other = __builtin_amdgcn_exp2f(mk - ts);
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll

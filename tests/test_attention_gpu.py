@@ -413,6 +413,20 @@ def test_fp32_ring_in_one_launch_each_way(b, sq, sk, d, P, dev):
     assert float((dq.cpu().double() - total).norm()) < 1e-5 * float(total.norm()) + floor
 
 
+@pytest.mark.parametrize("b", [3, 300, 520])  # 32, 64 and 128 rows a workgroup
+@pytest.mark.parametrize("dead", [(0, 32), (32, 64), (0, 70), (64, 70)])
+def test_fp32_steps_without_a_finite_score_weigh_nothing(b, dead, dev):
+    """Keys whose scores are all -inf, by whole steps of a wavefront or a whole chunk: the others' softmax, in whichever
+    group of wavefronts and at whichever place of the walk they fall (fp64 reference; the bar of the other fp32 tests)."""
+    torch.manual_seed(9)
+    q = torch.randn(b, 1, 33, 32).abs()
+    ks, vs = ([torch.randn(b, 1, 70, 32) for _ in range(2)] for _ in range(2))
+    ks[0][..., dead[0] : dead[1], :] = float("-inf")
+    want_o, want_l = oa.core_forward(q.double(), torch.cat(ks, -2).double(), torch.cat(vs, -2).double(), 0.125)
+    out, lse = ja._resident_forward(q.to(dev), [t.to(dev) for t in ks], [t.to(dev) for t in vs], 0.125)
+    assert rel_l2(out, want_o) < 1e-5 and rel_l2(lse, want_l) < 1e-5
+
+
 @pytest.mark.parametrize("d,n,nk", [(64, 192, 160), (32, 100, 70), (128, 64, 96)])
 def test_fp32_ring_step_takes_the_fused_merge(d, n, nk, dev):
     """``attend_step_`` on fp32 tensors at the head sizes of the fp32 matrix-core kernel: one launch that merges in
