@@ -41,6 +41,7 @@
 // Reference behaviour restated here:
 //   jigsaw/modules/attention/_functional/cores/math.py:125-149
 #include "attn_chunks.h"
+#include "lds_transfer.h"
 
 #include <type_traits>
 
@@ -71,25 +72,13 @@ __device__ __forceinline__ bf16x8 lds_frag(const unsigned char* p) {
   return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(p));
 }
 
-// One wavefront instruction lands 64 x 16 bytes contiguously in LDS, lane order = 8 rows: lane L
-// sits at row L / 8, chunk position L % 8 and fetches chunk (L % 8) ^ (row % 8) of its row.
-// Written in assembly: wave-uniform 64-bit source in scalar registers, the lane's constant
-// offset, the LDS address of the 1 KB block in M0. (With the compiler's own form of this load
-// it orders every later LDS read behind ALL outstanding transfers, also those of the tile
-// after next; the kernels order reads and transfers themselves, by their waits and barriers.)
-// the same for rows first_row + 0..7 of a tensor of `rows` rows, clamped to its last one
+// Offsets of a lane in a transfer of 8 rows (jg::to_lds_1k): lane L sits at row L / 8, chunk position L % 8 and
+// fetches chunk (L % 8) ^ (row % 8) of its row. First for rows first_row + 0..7 of a tensor of `rows` rows, clamped to its last one.
 __device__ __forceinline__ uint32_t dma_clamped_offset(int lane, int first_row, int rows) {
   return (uint32_t)min(first_row + (lane >> 3), rows - 1) * ROWB + (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4);
 }
 __device__ __forceinline__ uint32_t dma_lane_offset(int lane) {
   return (uint32_t)((lane >> 3) * ROWB + (((lane & 7) ^ (lane >> 3)) << 4));
-}
-__device__ __forceinline__ void dma_1k(const char* src, uint32_t lane_off, uint32_t lds_dst) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(src), "s"(lds_dst) : "m0");
-}
-__device__ __forceinline__ uint32_t lds_address(const unsigned char* p) {
-  typedef __attribute__((address_space(3))) unsigned char* lds_bytes;
-  return (uint32_t)(uintptr_t)((lds_bytes)p);
 }
 
 // fragment of a row-major tile: row r (0..63), 16-byte chunk c (0..7)
@@ -195,7 +184,7 @@ __global__ __launch_bounds__(DqPlan<QB>::THREADS, QB == 2 ? 2 : 1) void attn_bwd
   const char* kdma = chunk_entry(0, 0) + chunk_off;
   const char* vdma = chunk_entry(1, 0) + chunk_off;
   const uint32_t dma_off = dma_lane_offset(lane);
-  const uint32_t lds_dma = lds_address(smem) + (uint32_t)(ks_u * DqPlan<QB>::HALF + 16 * qb_u * ROWB);
+  const uint32_t lds_dma = jg::lds_address(smem) + (uint32_t)(ks_u * DqPlan<QB>::HALF + 16 * qb_u * ROWB);
   const int tr_off[2] = {tr_lane_offset(lane, 0), tr_lane_offset(lane, 1)};
   // row fragments: row ln of a 32-row block, chunk 2 c + kg
   int row_off[4];
@@ -208,16 +197,16 @@ __global__ __launch_bounds__(DqPlan<QB>::THREADS, QB == 2 ? 2 : 1) void attn_bwd
     const int row = row_first + ld_tile * DQ_BT;
     if (RAGGED) {
       const uint32_t o0 = dma_clamped_offset(lane, row, p.sk), o1 = dma_clamped_offset(lane, row + 8, p.sk);
-      dma_1k(kdma, o0, dst);
-      dma_1k(kdma, o1, dst + 8 * ROWB);
-      dma_1k(vdma, o0, dst + DQ_NAT);
-      dma_1k(vdma, o1, dst + DQ_NAT + 8 * ROWB);
+      jg::to_lds_1k(kdma, o0, dst);
+      jg::to_lds_1k(kdma, o1, dst + 8 * ROWB);
+      jg::to_lds_1k(vdma, o0, dst + DQ_NAT);
+      jg::to_lds_1k(vdma, o1, dst + DQ_NAT + 8 * ROWB);
     } else {
       const long long off = (long long)row * ROWB;
-      dma_1k(kdma + off, dma_off, dst);
-      dma_1k(kdma + off + 8 * ROWB, dma_off, dst + 8 * ROWB);
-      dma_1k(vdma + off, dma_off, dst + DQ_NAT);
-      dma_1k(vdma + off + 8 * ROWB, dma_off, dst + DQ_NAT + 8 * ROWB);
+      jg::to_lds_1k(kdma + off, dma_off, dst);
+      jg::to_lds_1k(kdma + off + 8 * ROWB, dma_off, dst + 8 * ROWB);
+      jg::to_lds_1k(vdma + off, dma_off, dst + DQ_NAT);
+      jg::to_lds_1k(vdma + off + 8 * ROWB, dma_off, dst + DQ_NAT + 8 * ROWB);
     }
     if (++ld_tile == tiles_per_chunk && ld_chunk + 1 < p.nchunks) {
       ld_tile = 0;
@@ -432,7 +421,7 @@ __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void at
   const char* qdma = reinterpret_cast<const char*>(p.q + b * p.sq * D);
   const char* ddma = reinterpret_cast<const char*>(p.dout + b * p.sq * D);
   const uint32_t dma_off = dma_lane_offset(lane);
-  const uint32_t lds_dma = lds_address(smem) + (uint32_t)(qs_u * (2 * DKV_HALF) + DKV_SHARE * kb_u * ROWB);
+  const uint32_t lds_dma = jg::lds_address(smem) + (uint32_t)(qs_u * (2 * DKV_HALF) + DKV_SHARE * kb_u * ROWB);
   const int tr_off[2] = {tr_lane_offset(lane, 0), tr_lane_offset(lane, 1)};
 
   float st_reg = 0.0f;
@@ -443,8 +432,8 @@ __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void at
       const int row = row_first + t * BT + r;
       const long long off = RAGGED ? 0 : (long long)row * ROWB;
       const uint32_t lane_off = RAGGED ? dma_clamped_offset(lane, row, p.sq) : dma_off;
-      dma_1k(qdma + off, lane_off, dst + r * ROWB);
-      dma_1k(ddma + off, lane_off, dst + NAT + r * ROWB);
+      jg::to_lds_1k(qdma + off, lane_off, dst + r * ROWB);
+      jg::to_lds_1k(ddma + off, lane_off, dst + NAT + r * ROWB);
     }
     // One plain load for every lane, used only when the statistics go to LDS: a load under a
     // per-lane condition, or arithmetic on its result here, would make the wavefront wait

@@ -44,6 +44,7 @@
 #include <initializer_list>
 
 #include "attn_chunks.h"
+#include "lds_transfer.h"
 
 namespace {
 
@@ -150,21 +151,13 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
   // contiguously in lane order = 8 rows; lane L sits at row L / 8, chunk position L % 8 and
   // fetches the chunk (L % 8) ^ (row % 8) of its row. A wavefront moves rows 16 qg .. 16 qg + 15
   // of the K tile and of the V tile (two instructions each).
-  // The transfer is written in assembly: a wave-uniform 64-bit base in scalar registers (tile
-  // and row block, advanced with scalar arithmetic), the lane's constant 32-bit offset, and the
-  // LDS address of the 1 KB block in M0, so that issuing a tile costs no vector instruction.
-  // (It also keeps the compiler from putting a wait for ALL outstanding transfers in front of
-  // every LDS read, which is how it orders LDS reads against transfers it knows about. The
-  // kernel orders them itself: a buffer is read only after the wait + barrier that follows its
-  // transfer, and refilled only after the barrier that follows its last read.)
+  // The base is wave-uniform (tile and row block, advanced with scalar arithmetic) and the lane's offset constant, so that
+  // issuing a tile costs no vector instruction (jg::to_lds_1k). A buffer is read only after the wait + barrier that
+  // follows its transfer, and refilled only after the barrier that follows its last read.
   const uint32_t dma_swz = (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4);
   const uint32_t dma_off = (uint32_t)((lane >> 3) * ROWB) + dma_swz;
   const int qg_u = __builtin_amdgcn_readfirstlane(qg), kq_u = __builtin_amdgcn_readfirstlane(kq);
-  typedef __attribute__((address_space(3))) unsigned char* lds_bytes;
-  const uint32_t lds_dma = (uint32_t)(uintptr_t)((lds_bytes)smem) + (uint32_t)(kq_u * QUARTER_BYTES + 16 * qg_u * ROWB);
-  auto dma_1k = [&](const char* src, uint32_t off, uint32_t dst) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(src), "s"(dst) : "m0");
-  };
+  const uint32_t lds_dma = jg::lds_address(smem) + (uint32_t)(kq_u * QUARTER_BYTES + 16 * qg_u * ROWB);
   // the load cursor: tiles are requested in stream order, the last one again and again past the end
   const long long chunk_off = 2 * (b * p.sk * (long long)D);  // bytes into a chunk
   const int row_first = kq_u * qtiles * BN + 16 * qg_u;       // the wavefront's first row in the quarter
@@ -174,10 +167,10 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
   auto dma_tile = [&](int buf) {
     const uint32_t dst = lds_dma + (uint32_t)(buf * TILE_BYTES);
     const long long off = (long long)(row_first + ld_tile * BN) * ROWB;
-    dma_1k(kdma + off, dma_off, dst);
-    dma_1k(kdma + off + 8 * ROWB, dma_off, dst + 8 * ROWB);
-    dma_1k(vdma + off, dma_off, dst + KV_BYTES);
-    dma_1k(vdma + off + 8 * ROWB, dma_off, dst + KV_BYTES + 8 * ROWB);
+    jg::to_lds_1k(kdma + off, dma_off, dst);
+    jg::to_lds_1k(kdma + off + 8 * ROWB, dma_off, dst + 8 * ROWB);
+    jg::to_lds_1k(vdma + off, dma_off, dst + KV_BYTES);
+    jg::to_lds_1k(vdma + off + 8 * ROWB, dma_off, dst + KV_BYTES + 8 * ROWB);
     if (ld_left > 0) {
       --ld_left;
       if (++ld_tile == qtiles) {
@@ -399,10 +392,10 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
       const uint32_t dst = lds_dma + (uint32_t)(buf * TILE_BYTES);
       const char* kc = chunk_entry(0, chunk) + chunk_off;
       const char* vc = chunk_entry(1, chunk) + chunk_off;
-      dma_1k(kc, o0, dst);
-      dma_1k(kc, o1, dst + 8 * ROWB);
-      dma_1k(vc, o0, dst + KV_BYTES);
-      dma_1k(vc, o1, dst + KV_BYTES + 8 * ROWB);
+      jg::to_lds_1k(kc, o0, dst);
+      jg::to_lds_1k(kc, o1, dst + 8 * ROWB);
+      jg::to_lds_1k(vc, o0, dst + KV_BYTES);
+      jg::to_lds_1k(vc, o1, dst + KV_BYTES + 8 * ROWB);
     };
     __syncthreads();  // every wavefront is past its last LDS read and its last transfer
     dma_tail(0, 0);

@@ -52,6 +52,7 @@
 #include <utility>
 
 #include "conv_common.h"
+#include "lds_transfer.h"
 
 namespace {
 
@@ -415,10 +416,9 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   // in registers of their own: no faster, and spills.) transfers_landed() before the barrier behind which they are read.
   auto load_weights = [&](int grp) {
     const char* const src = reinterpret_cast<const char*>(p.wprep + ((size_t)blockIdx.y * p.ngroups + grp) * w_slots);
-    typedef __attribute__((address_space(3))) unsigned char* lds_bytes;
-    const uint32_t lds_at = (uint32_t)(uintptr_t)(lds_bytes)smem;
+    const uint32_t lds_at = jg::lds_address(smem);
     for (int i = __builtin_amdgcn_readfirstlane(wave * 64); i < w_slots; i += THREADS)  // (64 divides the slots)
-      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"((uint32_t)(i + lane) * 16u), "s"(src), "s"(lds_at + (uint32_t)i * 16u) : "memory");
+      jg::to_lds_1k(src, (uint32_t)(i + lane) * 16u, lds_at + (uint32_t)i * 16u);
   };
   // The same from the weights as they are. raw_weights() puts the workgroup's share into the stage buffers (one run of memory
   // forward, a run for each contraction channel in the input gradient) and arrange_weights() deals it out from there, a slot of eight
@@ -432,13 +432,12 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   const int raw_len = p.transposed && runs == 1 ? p.C * run : run;  // elements of a run of memory
   auto raw_weights = [&]() {
     const uint16_t* const src = p.wraw + (size_t)mt * MT * taps_m * (p.transposed ? 1 : p.C);
-    typedef __attribute__((address_space(3))) unsigned char* lds_bytes;
-    const uint32_t lds_at = (uint32_t)(uintptr_t)(lds_bytes)lds_in;
+    const uint32_t lds_at = jg::lds_address(lds_in);
     const int per = raw_len / 8, pieces = runs * per;  // whole 16-byte pieces (with several runs a run is whole pieces: see the host)
     for (int i = __builtin_amdgcn_readfirstlane(wave * 64); i < pieces; i += THREADS) {
       const int at = min(i + lane, pieces - 1), r = runs == 1 ? 0 : at / per;
       const uint32_t off = 2u * (uint32_t)r * (uint32_t)(p.M * taps_m) + 16u * (uint32_t)(at - r * per);
-      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(src), "s"(lds_at + (uint32_t)i * 16u) : "memory");
+      jg::to_lds_1k(src, off, lds_at + (uint32_t)i * 16u);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();

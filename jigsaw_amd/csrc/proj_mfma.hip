@@ -24,6 +24,7 @@
 // proj_generic_kernel covers the other dtypes and unaligned shapes with plain FMAs.
 #include <type_traits>
 
+#include "lds_transfer.h"
 #include "reductions.h"
 
 namespace {
@@ -145,22 +146,7 @@ __device__ __forceinline__ u32x4 map8(u32x4 y, u32x4 r, F f) {
 }
 
 // ------------------------------------------------- memory -> LDS, both GEMMs
-// One wavefront instruction lands 64 x 16 bytes contiguously in LDS, in lane order; the source is a wave-uniform
-// base plus a 32-bit byte offset per lane (the host checks the tensor sizes), the LDS address of the 1 KB block goes
-// into M0. Written in assembly: with the compiler's own form it waits for ALL outstanding transfers before every
-// LDS read. The kernels order reads and transfers themselves, by one wait and one barrier per stage.
-__device__ __forceinline__ void dma_1k(const void* base, uint32_t lane_off, uint32_t lds_dst) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(base), "s"(lds_dst));
-}
-// The same for operands of 2^32 bytes and more: 64-bit offsets, added to the base lane by lane.
-__device__ __forceinline__ void dma_1k(const void* base, uint64_t lane_off, uint32_t lds_dst) {
-  const char* at = static_cast<const char*>(base) + lane_off;
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(at), "s"(lds_dst));
-}
-__device__ __forceinline__ uint32_t lds_address(const unsigned char* p) {
-  typedef __attribute__((address_space(3))) unsigned char* lds_bytes;
-  return (uint32_t)(uintptr_t)((lds_bytes)p);
-}
+// jg::to_lds_1k: 32-bit offsets where the host's check of the tensor sizes allows them, else 64-bit ones. One wait and one barrier per stage.
 __device__ __forceinline__ void transfers_landed() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // vmcnt(0)
 
 // Shape of a workgroup: WM x WN wavefronts, each with IM x JN blocks of 32 tokens x 32 features.
@@ -228,15 +214,15 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_nt_ke
     }
     if (p.bias != nullptr) bias_next = p.bias[min(n0 + tid, p.N - 1)];  // features past the end are dropped
   };
-  const uint32_t lds_a = lds_address(smem) + wave_u * 1024, lds_w = lds_a + SH::OP_A;
+  const uint32_t lds_a = jg::lds_address(smem) + wave_u * 1024, lds_w = lds_a + SH::OP_A;
   auto issue = [&](int buf) {
     const int k = ld_ks * BK + chunk * 8;
     const int kk = k < p.K ? k : 0;  // a chunk past the contraction length is read at k = 0 and zeroed below
     const uint32_t fa = (uint32_t)(feat_part(p.am, kk) * 2), fw = (uint32_t)kk * 2;
 #pragma unroll
-    for (int i = 0; i < SH::DMA_A; ++i) dma_1k(p.a, a_row[i] + fa, lds_a + buf * SH::STAGE + i * SH::WAVES * 1024);
+    for (int i = 0; i < SH::DMA_A; ++i) jg::to_lds_1k(p.a, a_row[i] + fa, lds_a + buf * SH::STAGE + i * SH::WAVES * 1024);
 #pragma unroll
-    for (int i = 0; i < SH::DMA_W; ++i) dma_1k(p.w, w_row[i] + fw, lds_w + buf * SH::STAGE + i * SH::WAVES * 1024);
+    for (int i = 0; i < SH::DMA_W; ++i) jg::to_lds_1k(p.w, w_row[i] + fw, lds_w + buf * SH::STAGE + i * SH::WAVES * 1024);
   };
   // the last stage of a contraction length that is no multiple of BK: a lane clears what its transfers put past it
   auto clear_tail = [&](int buf, int ks) {
@@ -490,7 +476,7 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
   TokenWalk<OFF> gw, xw;
   gw.start(p.gm, min(r_first + my_row, p.rows - 1));
   xw.start(p.xm, min(r_first + my_row, p.rows - 1));
-  const uint32_t lds_g = lds_address(smem) + wave_u * 1024;
+  const uint32_t lds_g = jg::lds_address(smem) + wave_u * 1024;
   auto issue = [&](int st, int buf) {
     const long long left = p.rows - (r_first + (long long)st * BR);
     const uint32_t dst = lds_g + buf * SH::STAGE;
@@ -498,8 +484,8 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
       TokenWalk<OFF> a = gw, b = xw;
 #pragma unroll
       for (int j = 0; j < SH::DMA; ++j) {
-        dma_1k(p.g, a.off + gf, dst + j * SH::WAVES * 1024);
-        dma_1k(p.x, b.off + xf, dst + SH::OP + j * SH::WAVES * 1024);
+        jg::to_lds_1k(p.g, a.off + gf, dst + j * SH::WAVES * 1024);
+        jg::to_lds_1k(p.x, b.off + xf, dst + SH::OP + j * SH::WAVES * 1024);
         a.advance(SH::JROWS);
         b.advance(SH::JROWS);
       }
@@ -509,8 +495,8 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
 #pragma unroll
       for (int j = 0; j < SH::DMA; ++j) {
         const long long r = min(r_first + (long long)st * BR + j * SH::JROWS + my_row, p.rows - 1);
-        dma_1k(p.g, (OFF)(row_part(p.gm, r) * 2) + gf, dst + j * SH::WAVES * 1024);
-        dma_1k(p.x, (OFF)(row_part(p.xm, r) * 2) + xf, dst + SH::OP + j * SH::WAVES * 1024);
+        jg::to_lds_1k(p.g, (OFF)(row_part(p.gm, r) * 2) + gf, dst + j * SH::WAVES * 1024);
+        jg::to_lds_1k(p.x, (OFF)(row_part(p.xm, r) * 2) + xf, dst + SH::OP + j * SH::WAVES * 1024);
       }
     }
   };
