@@ -284,11 +284,12 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_fwd_kernel(jg::ChunkTa
     }
   }
   if (!q_live) return;
-  const float inv = 1.0f / l;
-  const float lse_j = (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;  // v_log_f32 is log2
+  const bool none = l == 0.0f;  // no finite score: out 0, lse -inf, no weight in a merge (a score that is NaN makes l NaN)
+  const float inv = none ? 0.0f : 1.0f / l;
+  const float lse_j = none ? -INFINITY : (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;  // v_log_f32 is log2
   const long long qi = b * p.sq + qrow;
   float wt = 0.0f;
-  if (p.out_acc != nullptr) {
+  if (p.out_acc != nullptr && !none) {
     const float l_old = p.lse_acc[qi];
     wt = 1.0f / (1.0f + expf(l_old - lse_j));  // sigmoid(lse_j - l_old); l_old = -inf -> 1
     if (g == 0) p.lse_acc[qi] = fmaxf(l_old, lse_j) + log1pf(expf(-fabsf(l_old - lse_j)));

@@ -497,13 +497,14 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
   if (kq == 0) {
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-      const float inv = 1.0f / lt[qb];
-      const float lse_j = (m[qb] * c2 + log2f(lt[qb])) * 0.6931471805599453f;  // natural log
+      const bool none = lt[qb] == 0.0f;  // no finite score: out 0, lse -inf, no weight in a merge (a score that is NaN makes lt NaN)
+      const float inv = none ? 0.0f : 1.0f / lt[qb];
+      const float lse_j = none ? -INFINITY : (m[qb] * c2 + log2f(lt[qb])) * 0.6931471805599453f;  // natural log
       const int ql = qg * 64 + qb * 32 + ln;  // query inside the workgroup
       const long long qi = b * p.sq + where.blk * BM + ql;
       if (kg == 0 && (!RAGGED || where.blk * BM + ql < p.sq)) {
         float w = 0.0f;
-        if (p.out_acc != nullptr) {
+        if (p.out_acc != nullptr && !none) {
           const float l_old = p.lse_acc[qi];
           w = 1.0f / (1.0f + __expf(l_old - lse_j));  // sigmoid(lse_j - l_old); l_old = -inf -> 1
           const float mxl = fmaxf(l_old, lse_j);

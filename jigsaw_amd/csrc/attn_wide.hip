@@ -436,13 +436,14 @@ __global__ __launch_bounds__(64 * W * KS) void attn_wide_fwd_kernel(ChunkTable, 
     if (ks != 0) return;
   }
   if (!live) return;
-  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  const float lse_j = l > 0.0f ? m * p.scale + __logf(l) : -INFINITY;
+  const bool none = l == 0.0f;  // no finite score: out 0, lse -inf, no weight in a merge (a score that is NaN makes l NaN)
+  const float inv = none ? 0.0f : 1.0f / l;
+  const float lse_j = none ? -INFINITY : m * p.scale + __logf(l);
   const long long row = bh * p.sq + qi;
   // Ring merge (the reference's _online_softmax_merge_): w = sigmoid(lse_j - lse), out += w (out_j - out),
   // lse = logaddexp(lse, lse_j), with out_j rounded to the core's output dtype first as the unfused path has it.
   float w = 0.0f;
-  if (p.out_acc != nullptr) {
+  if (p.out_acc != nullptr && !none) {
     const float l_old = p.lse_acc[row];  // both lanes of the query read it before lane kg = 0 writes
     w = 1.0f / (1.0f + __expf(l_old - lse_j));  // l_old = -inf -> 1
     if (kg == 0) p.lse_acc[row] = fmaxf(l_old, lse_j) + log1pf(__expf(-fabsf(l_old - lse_j)));

@@ -57,7 +57,8 @@ __global__ __launch_bounds__(256) void merge_kernel(typename Elem<D1>::T* __rest
     }
     const float a = l1[l_off];
     const float b2 = l2[l_off];
-    const float w = 1.0f / (1.0f + __expf(a - b2));  // sigmoid(l2 - l1)
+    const bool none = b2 == -INFINITY;  // a part without a finite score weighs nothing, also beside an empty one
+    const float w = none ? 0.0f : 1.0f / (1.0f + __expf(a - b2));  // sigmoid(l2 - l1)
     struct alignas(sizeof(T1) * V) P1 { T1 v[V]; };
     struct alignas(sizeof(T2) * V) P2 { T2 v[V]; };
     P1 x = *reinterpret_cast<const P1*>(o1 + row * d + c);
@@ -71,7 +72,7 @@ __global__ __launch_bounds__(256) void merge_kernel(typename Elem<D1>::T* __rest
     *reinterpret_cast<P1*>(o1 + row * d + c) = x;
     if (c == 0) {
       const float mx = fmaxf(a, b2);
-      l_new[l_off] = mx + log1pf(__expf(-fabsf(a - b2)));
+      l_new[l_off] = none ? a : mx + log1pf(__expf(-fabsf(a - b2)));
     }
   }
 }

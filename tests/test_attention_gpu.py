@@ -427,6 +427,41 @@ def test_fp32_steps_without_a_finite_score_weigh_nothing(b, dead, dev):
     assert rel_l2(out, want_o) < 1e-5 and rel_l2(lse, want_l) < 1e-5
 
 
+@pytest.mark.parametrize("dtype,bar", [(torch.float32, 1e-5), (torch.bfloat16, 2e-2), (torch.float16, 4e-3)], ids=str)
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("b", [3, 300, 520])
+def test_a_chunk_without_a_finite_score_weighs_nothing_step_by_step(b, d, dtype, bar, dev):
+    """The same with the chunks arriving one by one, the dead one before, between and behind the others: the merge inside the
+    core's launch and the one of its own agree with the resident route. Where no key is left the row is 0 and its lse
+    -inf, and a NaN stays one."""
+    torch.manual_seed(9)
+    q = torch.randn(b, 1, 33, d).abs().to(dtype)
+    ks, vs = ([torch.randn(b, 1, 70, d).to(dtype) for _ in range(2)] for _ in range(2))
+    want_o, want_l = oa.core_forward(q.double(), torch.cat(ks, -2).double(), torch.cat(vs, -2).double(), 0.125)
+    q, dead, vd = q.to(dev), torch.full((b, 1, 70, d), float("-inf"), dtype=dtype, device=dev), torch.ones(b, 1, 70, d, dtype=dtype, device=dev)
+    live = [(k.to(dev), v.to(dev)) for k, v in zip(ks, vs)]
+    nothing = (torch.zeros(q.shape, device=dev), torch.full(q.shape[:-1], float("-inf"), device=dev))
+    merged = lambda k, v, out, lse: ja.fused_online_softmax_merge_(out, lse, *ja.core_forward(q, k, v, 0.125), "bhsd")  # noqa: E731
+    for step in (lambda k, v, out, lse: ja.attend_step_(q, k, v, 0.125, out, lse), merged):
+
+        def ring(chunks):
+            out, lse = (t.clone() for t in nothing)
+            for k, v in chunks:
+                out, lse = step(k, v, out, lse)
+            return out, lse
+
+        for at in range(3):
+            out, lse = ring([*live[:at], (dead, vd), *live[at:]])
+            assert rel_l2(out, want_o) < bar and rel_l2(lse, want_l) < bar
+        out, lse = ring([(dead, vd), (dead, vd)])
+        assert torch.equal(out, nothing[0]) and torch.equal(lse, nothing[1])
+        # a score that is NaN in the first row of the first entry
+        sick = live[0][0].clone()
+        sick[0, 0, 3, 1] = float("nan")
+        out, lse = ring([(sick, live[0][1]), live[1]])
+        assert out[0].isnan().all() and lse[0].isnan().all() and not out[1:].isnan().any() and not lse[1:].isnan().any()
+
+
 @pytest.mark.parametrize("d,n,nk", [(64, 192, 160), (32, 100, 70), (128, 64, 96)])
 def test_fp32_ring_step_takes_the_fused_merge(d, n, nk, dev):
     """``attend_step_`` on fp32 tensors at the head sizes of the fp32 matrix-core kernel: one launch that merges in
