@@ -151,8 +151,10 @@ def _as_64_columns(q, k, chunks: int = 1) -> bool:
     return rows <= 1 << 16
 
 
-def _padded_head_size(q, k, bias) -> int:
+def _padded_head_size(q, k, bias, want_dbias: bool = False) -> int:
     d = q.shape[-1]
+    if want_dbias:  # the gradient of a bias comes from the one-thread-per-row kernels, also where there is none to add
+        return _kernel_head_size(d, q.dtype, True)
     if bias is None and _mfma32(q, k):
         return (d + 3) // 4 * 4
     if not _mfma16(q, k, bias):
@@ -215,7 +217,7 @@ def core_backward(grad_out, q, k, v, out, logsumexp, scale, bias=None, want_dbia
     """``(dq, dk, dv[, dbias])`` of one chunk from the global ``out`` / ``logsumexp``."""
     _check_qkv(q, k, v)
     _lib.require_gpu(grad_out, out, logsumexp)
-    d, dp = q.shape[-1], _padded_head_size(q, k, bias)
+    d, dp = q.shape[-1], _padded_head_size(q, k, bias, want_dbias)
     if dp != d:
         res = _core_backward(_pad_last(grad_out, dp), _pad_last(q, dp), _pad_last(k, dp), _pad_last(v, dp),
                              _pad_last(out, dp), logsumexp, scale, bias, want_dbias)

@@ -413,6 +413,19 @@ def test_fp32_ring_in_one_launch_each_way(b, sq, sk, d, P, dev):
     assert float((dq.cpu().double() - total).norm()) < 1e-5 * float(total.norm()) + floor
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d", [4, 20, 32, 40, 96, 128])
+def test_gradient_of_a_bias_that_was_not_given(d, dtype, dev):
+    """``want_dbias`` without a bias at any head size: the gradient that a bias of zeros gets."""
+    torch.manual_seed(12)
+    q, k, v, dout = (torch.randn(2, 2, n, d, device=dev).to(dtype) for n in (37, 41, 41, 37))
+    out, lse = ja.core_forward(q, k, v, 0.125)
+    zeros = torch.zeros(2, 37, 41, device=dev)
+    for a, b in zip(ja.core_backward(dout, q, k, v, out, lse, 0.125, want_dbias=True),
+                    ja.core_backward(dout, q, k, v, out, lse, 0.125, bias=zeros, want_dbias=True)):
+        assert a.shape == b.shape and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("b", [3, 300, 520])  # 32, 64 and 128 rows a workgroup
 @pytest.mark.parametrize("dead", [(0, 32), (32, 64), (0, 70), (64, 70)])
 def test_fp32_steps_without_a_finite_score_weigh_nothing(b, dead, dev):
