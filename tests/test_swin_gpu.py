@@ -223,6 +223,28 @@ def test_sums_left_for_one_launch_have_the_bits_of_their_own(batch, n, dim, shif
     test_native_block_has_the_bits_of_the_python_route(batch, n, dim, shift, dev, monkeypatch)
 
 
+@pytest.mark.parametrize("batch,n,dim,shift", [(1, (128, 128), 128, 4), (2, (40, 56), 256, 0)])
+def test_native_backward_needs_no_more_memory_than_the_python_route(batch, n, dim, shift, dev, monkeypatch):
+    """The partials wait for their sums until the end; what else a backward makes and what the forward kept goes on the way."""
+    block = js.SwinBlock(dim, dim // 32, 8, n, shift=shift, device=dev)
+    x = torch.randn(batch, *n, dim, device=dev).bfloat16().requires_grad_()
+    g = torch.randn_like(x)
+
+    def peak():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = block(x)
+        torch.cuda.synchronize()
+        held = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        torch.autograd.grad(y, (x, *block.parameters()), g)
+        torch.cuda.synchronize()
+        return torch.cuda.max_memory_allocated() - held
+
+    native = peak()
+    monkeypatch.setattr(js._lib, "host", lambda: None)
+    assert native <= peak()
+
+
 @pytest.mark.parametrize("shift", [0, 4])
 def test_block_step_recorded_in_a_hip_graph_replays_the_eager_step(shift, dev):
     """``SwinBlock.captured_step``: forward + backward recorded once, replayed several times with eager
