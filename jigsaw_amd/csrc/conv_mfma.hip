@@ -1468,28 +1468,20 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     const int Hp = MODE == STRIDED_DGRAD ? p.Hx : p.Hout, Wp = MODE == STRIDED_DGRAD ? p.Wx : p.Wout;  // the produced tensor
     if (oh < 0 || oh >= Hp || ow < 0 || ow >= Wp) return;
     const uint32_t es = p.out_kind == 1 ? 4u : 2u;
-    char* base;
-    size_t ps, at;  // elements between channels of the destination, and to the pixel inside a channel
-    if (FOLD) {
-      auto region = [](int v, int lo, int n) { return v < lo ? 0 : (v < lo + n ? 1 : 2); };
-      auto within = [](int v, int r, int lo, int n) { return v - (r == 0 ? 0 : (r == 1 ? lo : lo + n)); };
-      auto extent = [](int r, int lo, int n, int all) { return r == 0 ? lo : (r == 1 ? n : all - lo - n); };
-      const int rd = region(tc.od, p.lo_d, p.nD), rh = region(oh, p.lo_h, p.nH), rw = region(ow, p.lo_w, p.nW);
-      // (wave-uniform indices into the table: see epilogue_fold)
-      constexpr int STEP = ALONG_H ? 3 : 1;
-      const int slot = __builtin_amdgcn_readfirstlane(rd * 9 + (ALONG_H ? rw : 3 * rh)), r = ALONG_H ? rh : rw;
-      char* const low = static_cast<char*>(strip_entry(slot));
-      char* const mid = slot + STEP == 13 ? reinterpret_cast<char*>(p.y) : static_cast<char*>(strip_entry(slot + STEP));
-      char* const high = static_cast<char*>(strip_entry(slot + 2 * STEP));
-      base = r == 0 ? low : (r == 1 ? mid : high);
-      const int eh = extent(rh, p.lo_h, p.nH, Hp), ew = extent(rw, p.lo_w, p.nW, Wp);
-      ps = (size_t)extent(rd, p.lo_d, p.nD, p.Dout) * eh * ew;
-      at = ((size_t)within(tc.od, rd, p.lo_d, p.nD) * eh + within(oh, rh, p.lo_h, p.nH)) * ew + within(ow, rw, p.lo_w, p.nW);
-    } else {
-      base = reinterpret_cast<char*>(p.y);
-      ps = (size_t)p.Dout * Hp * Wp;
-      at = ((size_t)tc.od * Hp + oh) * Wp + ow;
-    }
+    auto region = [](int v, int lo, int n) { return v < lo ? 0 : (v < lo + n ? 1 : 2); };
+    auto within = [](int v, int r, int lo, int n) { return v - (r == 0 ? 0 : (r == 1 ? lo : lo + n)); };
+    auto extent = [](int r, int lo, int n, int all) { return r == 0 ? lo : (r == 1 ? n : all - lo - n); };
+    const int rd = region(tc.od, p.lo_d, p.nD), rh = region(oh, p.lo_h, p.nH), rw = region(ow, p.lo_w, p.nW);
+    // (wave-uniform indices into the table: see epilogue_fold)
+    constexpr int STEP = ALONG_H ? 3 : 1;
+    const int slot = __builtin_amdgcn_readfirstlane(rd * 9 + (ALONG_H ? rw : 3 * rh)), r = ALONG_H ? rh : rw;
+    char* const low = static_cast<char*>(strip_entry(slot));
+    char* const mid = slot + STEP == 13 ? reinterpret_cast<char*>(p.y) : static_cast<char*>(strip_entry(slot + STEP));
+    char* const high = static_cast<char*>(strip_entry(slot + 2 * STEP));
+    char* const base = r == 0 ? low : (r == 1 ? mid : high);
+    const int eh = extent(rh, p.lo_h, p.nH, Hp), ew = extent(rw, p.lo_w, p.nW, Wp);
+    const size_t ps = (size_t)extent(rd, p.lo_d, p.nD, p.Dout) * eh * ew;  // elements between channels of the destination
+    const size_t at = ((size_t)within(tc.od, rd, p.lo_d, p.nD) * eh + within(oh, rh, p.lo_h, p.nH)) * ew + within(ow, rw, p.lo_w, p.nW);
     if (base == nullptr) return;
     const uintptr_t to = reinterpret_cast<uintptr_t>(base) + es * (((size_t)tc.n * p.M + m0) * ps + at);
 #pragma unroll
@@ -1498,10 +1490,10 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
       const uintptr_t d = to + es * ps * channel(i);
       const float v = value(i);
       if (p.out_kind == 1) {
-        *reinterpret_cast<JG_GLOBAL float*>(d) = FOLD ? 0.0f + v : v;  // (a sum with zero clears a zero's sign)
+        *reinterpret_cast<JG_GLOBAL float*>(d) = 0.0f + v;  // (a sum with zero clears a zero's sign)
       } else {
         uint16_t bits = F16 ? __builtin_bit_cast(uint16_t, (_Float16)v) : __builtin_bit_cast(uint16_t, (__bf16)v);
-        if (FOLD && (bits & 0x7fffu) == 0) bits = 0;
+        if ((bits & 0x7fffu) == 0) bits = 0;
         *reinterpret_cast<JG_GLOBAL uint16_t*>(d) = bits;
       }
     }
