@@ -533,9 +533,8 @@ static int swin_bwd(const char* who, jg_reductions* later, void* dq, void* dk, v
   a.lse = const_cast<float*>(lse);
   a.bins = static_cast<float*>(workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // As many wavefronts as the device holds at a time (256 compute units, two workgroups each by LDS),
-  // the same number for every head.
-  const long long windows = a.entries / heads, most = (512ll * WAVES) / heads;
+  // As many wavefronts as the device holds at a time (two workgroups a compute unit by LDS), the same number for every head.
+  const long long windows = a.entries / heads, most = 2ll * jg::cu_count() * WAVES / heads;
   a.slots = (int)(most < 1 ? 1 : windows < most ? windows : most);
   const long long workers = (long long)a.slots * heads;
   const dim3 grid((unsigned)((workers + WAVES - 1) / WAVES));
