@@ -6,6 +6,7 @@ import itertools
 
 import torch
 
+from jigsaw_amd import _lib
 from jigsaw_amd.halo import HaloGeometry
 
 
@@ -29,6 +30,26 @@ def rel_l2(got: torch.Tensor, want: torch.Tensor) -> float:
     w = want.detach().double().cpu()
     den = w.norm().item()
     return (g - w).norm().item() / (den if den > 0 else 1.0)
+
+
+def native_answers(monkeypatch, *names) -> dict:
+    """How often each of these functions of the native host module has returned a result from here on (instead of ``None``, with which it
+    leaves a call to the Python route)."""
+    host = _lib.host()
+    assert host is not None, "the native host module is not built"
+    counts = dict.fromkeys(names, 0)
+
+    def counted(name, call):
+        def answer(*args):
+            got = call(*args)
+            counts[name] += got is not None
+            return got
+
+        return answer
+
+    for name in names:
+        monkeypatch.setattr(host, name, counted(name, getattr(host, name)))
+    return counts
 
 
 def mesh_coords(mesh_shape):

@@ -17,6 +17,10 @@ pytestmark = pytest.mark.gpu
 TOL = {torch.float32: 1e-5, torch.bfloat16: 2e-2, torch.float16: 2e-2}
 
 
+def _compute_units() -> int:
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
 def _qkv(b, h, sq, sk, d, dtype, seed=0):
     torch.manual_seed(seed)
     q = (torch.randn(b, h, sq, d) / d**0.5).to(dtype)
@@ -29,14 +33,16 @@ CORE_SHAPES = [
     (3, 6, 64, 64, 16),   # the reference's ring test shape per chunk (b=3, h=6, n=16*4, d=16)
     (2, 2, 50, 70, 32),   # ragged
     (1, 3, 130, 33, 64),
-    (1, 2, 128, 128, 64),  # MFMA path for bf16
-    (2, 2, 256, 384, 64),  # MFMA path for bf16
+    (1, 2, 128, 128, 64),  # MFMA path for bf16; few workgroups of 64 queries: the kernel of any head size
+    (2, 2, 256, 384, 64),  # the same
+    (1, 70, 256, 384, 64),  # the forward kernel of head size 64
     (1, 1, 40, 40, 128),
     (1, 2, 17, 9, 8),
     (1, 3, 256, 128, 32),  # head sizes below 64: kernels of 32 and 64 columns
     (2, 2, 128, 256, 16),
     (1, 2, 200, 300, 32),  # ragged queries and keys below head size 64
-    (1, 2, 130, 260, 64),  # ragged at head size 64: 256 keys in the pipeline, 4 behind it
+    (1, 2, 130, 260, 64),  # ragged at head size 64
+    (1, 100, 130, 260, 64),  # and in its own forward kernel: 256 keys in the pipeline, 4 behind it
     (2, 1, 128, 130, 16),
     (1, 1, 70, 1000, 64),
     (1, 2, 128, 256, 128),  # head sizes 96 and 128: their own MFMA kernels for bf16
@@ -177,15 +183,17 @@ def test_fp32_head_sizes_between_the_matrix_core_sizes(d, dev):
         assert got.shape == want.shape and rel_l2(got, want) < 1e-5
 
 
+@pytest.mark.parametrize("h", [2, 70], ids=["kernel of any head size", "kernel of head size 64"])
 @pytest.mark.parametrize("pattern", ["late_spike", "rising", "first_tile_low", "huge_logits", "one_hot_rows"])
-def test_mfma_forward_when_the_running_max_moves(pattern, dev):
-    """The head-size-64 kernel keeps a per-query reference exponent that follows the running
+def test_mfma_forward_when_the_running_max_moves(pattern, h, dev):
+    """Launches of few workgroups of 64 queries run the kernel of any head size; the head-size-64 kernel keeps a per-query reference exponent that follows the running
     max lazily (it moves only when a tile exceeds it by 2^8) and folds it into the score
     product. Score patterns that move the max late, often, by hundreds of powers of two, or
     start far below zero must give the fp64 softmax all the same (bf16 bar), and so must
     the merge into a ring accumulator that already holds a chunk."""
     torch.manual_seed(11)
-    b, h, sq, sk, d = 1, 2, 256, 1024, 64
+    b, sq, sk, d = 1, 256, 1024, 64
+    assert (h * (sq // 64) > _compute_units()) == (h == 70)
     q = torch.randn(b, h, sq, d)
     k = torch.randn(b, h, sk, d)
     v = torch.randn(b, h, sk, d)
@@ -354,11 +362,12 @@ def test_backward_over_resident_chunks_in_one_pass(b, h, n, nk, P, dev):
     assert torch.equal(dq2, dq) and all(torch.equal(a, c) for a, c in zip(dks2, dks))
 
 
-@pytest.mark.parametrize("heads", [2, 150], ids=["64-query workgroups", "128-query workgroups"])
+@pytest.mark.parametrize("heads", [2, 150], ids=["32-query workgroups", "128-query workgroups"])
 @pytest.mark.parametrize("n,nk,P", [(64, 128, 1), (65, 129, 1), (128, 192, 1), (127, 257, 1), (33, 320, 1), (96, 383, 1), (130, 448, 1), (64, 640, 1), (100, 1100, 1),
                                     (64, 128, 2), (70, 190, 3), (128, 256, 5)], ids=str)
 def test_query_gradient_at_the_ends_of_its_key_tiles(heads, n, nk, P, dev):
-    """One to eighteen tiles of a key half (four a round, then one by one), chunks that end inside a tile, both workgroup sizes. dS is rounded to bf16,
+    """One to eighteen tiles of a key half (four a round, then one by one), chunks that end inside a tile, workgroups of 32 queries (the kernel
+    of any head size) and of 128. dS is rounded to bf16,
     half of 2^-8, and so is the result; twice that leaves room for the exponential and the sums."""
     torch.manual_seed(n + nk)
     d, scale = 64, 0.125
@@ -370,6 +379,15 @@ def test_query_gradient_at_the_ends_of_its_key_tiles(heads, n, nk, P, dev):
     dS = torch.exp(Q @ K.mT * scale - L[..., None]) * (dO @ V.mT - (dO * O).sum(-1, keepdim=True)) * scale
     off = (dq[0].double().cpu() - dS @ K).abs() - 2.0**-8 * (dS.abs() @ K.abs() + (dS @ K).abs())
     assert off.max() <= 0, off.max()
+
+
+@pytest.mark.parametrize("heads,n,nk,P", [(100, 65, 129, 1), (100, 96, 383, 1), (100, 127, 257, 1), (100, 128, 192, 1), (100, 128, 640, 1), (100, 128, 256, 5),
+                                          (100, 70, 190, 3), (60, 130, 448, 1), (60, 150, 1100, 2), (60, 192, 128, 1)], ids=str)
+def test_query_gradient_in_workgroups_of_64_queries(heads, n, nk, P, dev):
+    """The same between the two: enough rows for workgroups of 32 to fill the chip, too few for those of 128 to do so."""
+    cus = _compute_units()
+    assert heads * -(-n // 32) > cus and 2 * heads * -(-n // 128) <= cus
+    test_query_gradient_at_the_ends_of_its_key_tiles(heads, n, nk, P, dev)
 
 
 def test_backward_over_chunks_declines_what_it_does_not_cover(dev):
@@ -670,6 +688,8 @@ def test_short_key_ranges_keep_probabilities_in_fp32(h, sq, sk, d, P, dtype, dev
 @pytest.mark.parametrize("h,sq,sk,d,P,dtype", [
     (3, 130, 300, 64, 1, torch.bfloat16), (3, 256, 1000, 64, 3, torch.bfloat16), (30, 256, 1000, 128, 2, torch.bfloat16),
     (3, 130, 255, 96, 3, torch.bfloat16), (30, 256, 1000, 128, 2, torch.float16), (3, 130, 255, 96, 3, torch.float16),
+    # workgroups of 128 queries, at bf16 and head size 64 the kernel of that size
+    (100, 130, 300, 64, 1, torch.bfloat16), (70, 256, 1000, 64, 3, torch.bfloat16), (70, 256, 1000, 128, 2, torch.bfloat16), (100, 130, 255, 96, 3, torch.float16),
 ], ids=str)
 def test_keys_behind_the_last_whole_tile_keep_probabilities_in_fp32(h, sq, sk, d, P, dtype, dev):
     """Forward at a head size that fills a kernel: the keys of a chunk behind its last multiple of 128. The whole tiles
@@ -685,11 +705,12 @@ def test_keys_behind_the_last_whole_tile_keep_probabilities_in_fp32(h, sq, sk, d
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("h", [2, 140], ids=["workgroups of 32 queries", "workgroups of 128 queries"])
 @pytest.mark.parametrize("sq,sk,d", [(70, 100, 64), (70, 1000, 64), (70, 100, 128), (70, 200, 96), (70, 33, 32)], ids=str)
-def test_infinite_values_stay_infinite_where_probabilities_are_kept_in_fp32(sq, sk, d, dtype, dev):
+def test_infinite_values_stay_infinite_where_probabilities_are_kept_in_fp32(sq, sk, d, h, dtype, dev):
     """A value that is infinite makes its output column infinite, not NaN, also as the last key of a range."""
     torch.manual_seed(sk)
-    q, k, v = (torch.randn(1, 2, n, d, device=dev).to(dtype) for n in (sq, sk, sk))
+    q, k, v = (torch.randn(1, h, n, d, device=dev).to(dtype) for n in (sq, sk, sk))
     v[..., sk - 1, 3], v[..., sk // 2, 5] = float("inf"), float("-inf")
     out, _ = ja.core_forward(q, k, v, d**-0.5)
     want, _ = ja.core_forward(q, k, v, d**-0.5, bias=torch.zeros(sq, sk, device=dev))

@@ -8,7 +8,7 @@ checked exactly: with a one-hot weight the projection is a pure copy.
 import pytest
 import torch
 
-from helpers import rel_l2
+from helpers import native_answers, rel_l2
 from jigsaw_amd import projection as jp
 from oracle import projection as op
 
@@ -93,6 +93,7 @@ def test_native_projections_have_the_bits_of_the_python_route(case, need, dev, m
     make = lambda *shape: torch.randn(*shape, device=dev, generator=gen).to(dtype)  # noqa: E731
     x, w, b, g = make(*lead, s, c), make(3 * heads * d, c), make(3 * heads * d), make(3, *lead, heads, s, d)
     o, wo, bo, g2 = make(*lead, heads, s, d), make(n2, heads * d), make(n2), make(*lead, s, n2)
+    answers = native_answers(monkeypatch, "qkv_forward", "heads_forward", "projection_backward")
 
     def passes():
         out = []
@@ -108,6 +109,8 @@ def test_native_projections_have_the_bits_of_the_python_route(case, need, dev, m
         return out
 
     here = passes()
+    some, wanted = int(x.numel() > 0), need[0] or need[1] or (need[2] and has_b)  # an empty batch is the Python route's
+    assert answers == {"qkv_forward": some, "heads_forward": some, "projection_backward": 2 * some * wanted}
     monkeypatch.setattr(jp._lib, "host", lambda: None)
     for a, want in zip(here, passes()):
         assert (a is None and want is None) or torch.equal(a, want)

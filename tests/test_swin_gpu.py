@@ -12,7 +12,7 @@ tests/test_examples.py:48-67); rel-L2 2e-2 in bf16.
 import pytest
 import torch
 
-from helpers import mesh_coords, rel_l2
+from helpers import mesh_coords, native_answers, rel_l2
 from jigsaw_amd import swin as js
 from jigsaw_amd.conv import TileGroup
 from oracle import roll as orl
@@ -191,7 +191,8 @@ def test_block_as_one_autograd_node_has_the_bits_of_its_parts(shift, n, dev):
 
 @pytest.mark.parametrize("batch,n,dim,shift", [(1, (8, 8), 64, 4), (2, (24, 40), 96, 0), (3, (32, 16), 256, 3)])
 def test_native_block_has_the_bits_of_the_python_route(batch, n, dim, shift, dev, monkeypatch):
-    """A gradient off the 16-byte grid and a pass without any gradient among them."""
+    """A gradient off the 16-byte grid and a pass without any gradient among them. (A backward of a native pass that declined would raise.)"""
+    answers = native_answers(monkeypatch, "swin_forward")
     torch.manual_seed(6)
     block = js.SwinBlock(dim, dim // 32, 8, n, shift=shift, device=dev)
     x = torch.randn(batch, *n, dim, device=dev).bfloat16()
@@ -209,6 +210,7 @@ def test_native_block_has_the_bits_of_the_python_route(batch, n, dim, shift, dev
         xg = x.clone().requires_grad_()
         off = torch.autograd.grad(block(xg), (xg, *block.parameters()), g)
     here = passes()
+    assert answers == {"swin_forward": 3}
     for a, want in zip(off, here[2:]):
         assert torch.equal(a, want)
     monkeypatch.setattr(js._lib, "host", lambda: None)
@@ -226,6 +228,7 @@ def test_sums_left_for_one_launch_have_the_bits_of_their_own(batch, n, dim, shif
 @pytest.mark.parametrize("batch,n,dim,shift", [(1, (128, 128), 128, 4), (2, (40, 56), 256, 0)])
 def test_native_backward_needs_no_more_memory_than_the_python_route(batch, n, dim, shift, dev, monkeypatch):
     """The partials wait for their sums until the end; what else a backward makes and what the forward kept goes on the way."""
+    answers = native_answers(monkeypatch, "swin_forward")
     block = js.SwinBlock(dim, dim // 32, 8, n, shift=shift, device=dev)
     x = torch.randn(batch, *n, dim, device=dev).bfloat16().requires_grad_()
     g = torch.randn_like(x)
@@ -241,6 +244,7 @@ def test_native_backward_needs_no_more_memory_than_the_python_route(batch, n, di
         return torch.cuda.max_memory_allocated() - held
 
     native = peak()
+    assert answers == {"swin_forward": 1}
     monkeypatch.setattr(js._lib, "host", lambda: None)
     assert native <= peak()
 
