@@ -154,6 +154,31 @@ __device__ __forceinline__ void clear_acc(f32x16 (&acc)[NT]) {
     for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
 }
 
+// acc = acc * mul + A^T B over the 32 rows of a step: `rows` (LDS) holds A as rows of PITCH floats, of which this lane takes column 32 t + n; b
+// is the other operand as it lies in the registers. The matrix cores sum a step from zero and the vector unit adds it to the steps before:
+// output and dQ are sums over the keys of all chunks, which in the matrix cores' accumulators alone are one chain of roundings. Relative errors
+// of the output and dQ, 64 heads x 1000 x 16 chunks at 64: one chain 2.3e-6 / 2.3e-6, a launch and a chain a chunk 8.3e-7 / 7.5e-7, this
+// 6.1e-7 / 6.3e-7; 16 x 64 x 8 chunks 3.6e-7 / 3.9e-7 a chunk, this 2.5e-7 / 3.8e-7. It costs 1 to 3 % at widths up to 96 (16 x 700 x 4 at
+// 64 491 -> 503 us both ways) and gains 4 % at 128, whose accumulators no longer wait for the factor (48 x 900 x 4 4864 -> 4668).
+template <int NT, int PITCH>
+__device__ __forceinline__ void add_step(f32x16 (&acc)[NT], const float* rows, const f32x16& b, int g, float mul) {
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    f32x16 sum;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sum[i] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(rows[row_of(i, g) * PITCH + 32 * t], b[i], sum, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[t][i] = acc[t][i] * mul + sum[i];
+  }
+}
+
+// Wavefronts a SIMD that the two kernels are held to where the compiler would take a few registers more than leave room for them: 64 heads x 1000 x 3
+// chunks at 96 3162 -> 3030 us, x 4 at 32 1533 -> 1498.
+constexpr int fwd_waves(int D, int R) { return D == 32 ? (R == 1 ? 3 : 4) : D == 64 || (D == 96 && R == 4) ? 2 : 1; }
+constexpr int dq_waves(int D, int R) { return D == 32 ? (R == 4 ? 4 : 3) : (D == 64 && R > 1) || (D == 96 && R == 4) ? 2 : 1; }
+
 struct F32Params {
   const float* q;      // (batch, sq, d)
   float* out;          // (batch, sq, d) or NULL
@@ -165,7 +190,7 @@ struct F32Params {
 };
 
 template <int D, int R>
-__global__ __launch_bounds__(kThreads) void attn_f32_mfma_fwd_kernel(jg::ChunkTable, F32Params p) {
+__global__ __launch_bounds__(kThreads, fwd_waves(D, R)) void attn_f32_mfma_fwd_kernel(jg::ChunkTable, F32Params p) {
   typedef Shape<D, R> S;
   constexpr int H = S::H, PITCH = S::PITCH, NT = S::NT, G = S::G;
   extern __shared__ __attribute__((aligned(16))) float smem[];
@@ -242,18 +267,7 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_fwd_kernel(jg::ChunkTa
     sum += __shfl_xor(sum, 32, 64);
     l = l * alpha + sum;
     m = m_new;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) o[t][i] *= alpha;
-
-    // O^T[dv][query] += V^T P^T
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float* vrow = Vs + row_of(i, g) * PITCH + n;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 * t], s[i], o[t], 0, 0, 0);
-    }
+    add_step<NT, PITCH>(o, Vs + n, s, g, alpha);  // O^T[dv][query] += V^T P^T
   }
 
   if (G > 1) {  // the groups' results by their maxima, in the order of the groups
@@ -286,7 +300,7 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_fwd_kernel(jg::ChunkTa
   if (!q_live) return;
   const bool none = l == 0.0f;  // no finite score: out 0, lse -inf, no weight in a merge (a score that is NaN makes l NaN)
   const float inv = none ? 0.0f : 1.0f / l;
-  const float lse_j = none ? -INFINITY : (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;  // v_log_f32 is log2
+  const float lse_j = none ? -INFINITY : fmaf(m, 0.6931471805599453f, __builtin_amdgcn_logf(l) * 0.6931471805599453f);  // v_log_f32 is log2
   const long long qi = b * p.sq + qrow;
   float wt = 0.0f;
   if (p.out_acc != nullptr && !none) {
@@ -350,7 +364,7 @@ __device__ __forceinline__ void store_rows(float* row, const f32x16 (&acc)[NT], 
 }
 
 template <int D, int R>
-__global__ __launch_bounds__(kThreads) void attn_f32_mfma_dq_kernel(jg::ChunkTable, F32BwdParams p) {
+__global__ __launch_bounds__(kThreads, dq_waves(D, R)) void attn_f32_mfma_dq_kernel(jg::ChunkTable, F32BwdParams p) {
   typedef Shape<D, R> S;
   constexpr int H = S::H, PITCH = S::PITCH, NT = S::NT, G = S::G;
   extern __shared__ __attribute__((aligned(16))) float smem[];
@@ -430,12 +444,7 @@ __global__ __launch_bounds__(kThreads) void attn_f32_mfma_dq_kernel(jg::ChunkTab
       if (ragged && key0 + row_of(i, g) >= p.sk) pr = 0.0f;
       s[i] = pr * (dp[i] - dl);  // dS^T
     }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float* krow = Ks + row_of(i, g) * PITCH + n;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) dq[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(krow[32 * t], s[i], dq[t], 0, 0, 0);
-    }
+    add_step<NT, PITCH>(dq, Ks + n, s, g, 1.0f);
   }
   if (G > 1) {
     constexpr int PART = NT * 16 * 64;
