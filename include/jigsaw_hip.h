@@ -625,7 +625,8 @@ int jg_bias_grad(void* gb, const void* g, int64_t batch, int64_t channels,
  * which is _online_softmax_merge_ (forward.py:23-61) without the round trip of
  * out_j through HBM; `out` / `lse` may then be NULL (bf16 and fp16 with d a multiple of 8
  * up to 128, fp32 with d a multiple of 4 up to 128; no bias, 16-byte aligned tensors, any sq and sk;
- * JG_ERR_UNSUPPORTED otherwise).
+ * JG_ERR_UNSUPPORTED otherwise). A row whose scores are all -inf gives out 0 and lse -inf there and
+ * changes nothing where it is merged (jg_lse_merge does the same with a part whose lse is -inf).
  * Without a bias and with 16-byte aligned tensors those types and head sizes run on the
  * matrix cores (forward and backward). Everything else runs on one-thread-per-row kernels,
  * which take any alignment and d = 8, 16, 32, 64, 96, 128 (JG_ERR_UNSUPPORTED otherwise;

@@ -634,7 +634,7 @@ int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
   // Where even those of 64 would leave half of them without one, 32 queries and eight key groups (attn_width; this kernel with 64 : that one, us):
   // 1 x 8 heads x 1024 x 8 chunks 73 : 52, 1 x 8 x 512 x 4 20.8 : 18.0, 2 x 4096 x 2 70 : 52, 4 x 1024 x 1 12.2 : 12.4.
   // Where workgroups of 128 queries would leave half of the compute units without one, those of 64 queries (128 : 64, us): 8 heads x
-  // 2048 queries x 4 chunks 94 : 81, 3 x 4000 x 8 321 : 285, 18 x 700 x 3 32 : 26, 10 x 284 x 3 19 : 13. Elsewhere twice the tile
+  // 2048 queries x 4 chunks 94 : 81, 3 x 4000 x 8 321 : 285, 18 x 700 x 3 32 : 26. Elsewhere twice the tile
   // traffic and a barrier for half the keys cost more than the waves' independence gives: 8 x 4096 x 4 203 : 223, 32 x 1024 x 1
   // 18.0 : 18.9, 24 x 1000 x 2 30.8 : 32.1.
   if (attn_width(sq, batch, D) == 1) {

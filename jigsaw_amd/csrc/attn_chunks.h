@@ -83,11 +83,10 @@ __device__ __forceinline__ void parts8(const float* v, bf16x8_t (&part)[3]) {
 // Wavefronts of 32 rows each that share a tile of the streamed side in the kernels of attn_wide.hip: four, or as many fewer as it takes
 // to give every compute unit a workgroup. A tile takes 1.3 to 2.5 us of latency whatever else runs there (fetch, scores, exponentials,
 // products, one after the other), so that 48 workgroups of 128 rows left the chip idle for as long as a full one; with 64 or 32 rows they
-// are two or four times as many, and what their fewer rows leave free takes more tiles at once (four to eight groups a workgroup). Forward / backward,
-// us, before -> with it: 1 x 8 heads x 512 x 4 chunks, head size 128 47 / 84 -> 32 / 59, fp16 64 29 / 46 -> 17 / 30, 8 chunks at 32 39 / 59 -> 19 / 32;
-// 4 x 1006 x 5, 80 92 / 124 -> 53 / 83; 2 x 197 x 5, fp16 96 47 / 41 -> 24 / 26. Forced, where 128 rows have a workgroup for every second
-// compute unit or more: 60 x 529 x 4, fp16 96 94 / 190 -> 125 / 209 (64 rows); at head size 32, whose workgroups fit a compute unit several times,
-// up to two of 64 rows each still gain: 28 x 931 x 7 84 / 156 -> 78 / 152, 14 x 1442 x 5 87 / 153 -> 77 / 139.
+// are two or four times as many, and what their fewer rows leave free takes more tiles at once (four to eight groups a workgroup).
+// Forward / backward, us, before -> with it: 8 heads x 512 x 4 chunks at 128 47 / 84 -> 31 / 59, x 8 chunks at 32 39 / 59 -> 19 / 29. Forced, where 128 rows
+// have a workgroup for every second compute unit or more: 60 x 529 x 4, fp16 96 94 / 190 -> 125 / 209 (64 rows). At head size 32, whose workgroups
+// fit a compute unit several times, up to two of 64 rows each still gain: 28 x 931 x 7 84 / 156 -> 78 / 152.
 inline int attn_width(long long rows, long long batch, int columns) {
   if (cdiv(rows, 32) * batch <= cu_count()) return 1;
   return cdiv(rows, 64) * batch <= (columns == 32 ? 2 : 1) * cu_count() ? 2 : 4;

@@ -159,7 +159,7 @@ __device__ __forceinline__ void clear_acc(f32x16 (&acc)[NT]) {
 // output and dQ are sums over the keys of all chunks, which in the matrix cores' accumulators alone are one chain of roundings. Relative errors
 // of the output and dQ, 64 heads x 1000 x 16 chunks at 64: one chain 2.3e-6 / 2.3e-6, a launch and a chain a chunk 8.3e-7 / 7.5e-7, this
 // 6.1e-7 / 6.3e-7; 16 x 64 x 8 chunks 3.6e-7 / 3.9e-7 a chunk, this 2.5e-7 / 3.8e-7. It costs 1 to 3 % at widths up to 96 (16 x 700 x 4 at
-// 64 491 -> 503 us both ways) and gains 4 % at 128, whose accumulators no longer wait for the factor (48 x 900 x 4 4864 -> 4668).
+// 64 489 -> 501 us both ways) and gains 3 to 5 % at 128, whose accumulators no longer wait for the factor (48 x 900 x 4 4871 -> 4641).
 template <int NT, int PITCH>
 __device__ __forceinline__ void add_step(f32x16 (&acc)[NT], const float* rows, const f32x16& b, int g, float mul) {
 #pragma unroll
@@ -175,7 +175,7 @@ __device__ __forceinline__ void add_step(f32x16 (&acc)[NT], const float* rows, c
 }
 
 // Wavefronts a SIMD that the two kernels are held to where the compiler would take a few registers more than leave room for them: 64 heads x 1000 x 3
-// chunks at 96 3162 -> 3030 us, x 4 at 32 1533 -> 1498.
+// chunks at 96 3162 -> 3018 us, x 4 at 32 1533 -> 1491.
 constexpr int fwd_waves(int D, int R) { return D == 32 ? (R == 1 ? 3 : 4) : D == 64 || (D == 96 && R == 4) ? 2 : 1; }
 constexpr int dq_waves(int D, int R) { return D == 32 ? (R == 4 ? 4 : 3) : (D == 64 && R > 1) || (D == 96 && R == 4) ? 2 : 1; }
 
@@ -588,10 +588,10 @@ bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15)
 // Resident rows of a workgroup, in wavefronts: what the busiest compute unit has to do (its workgroups, each R / 4 of the
 // streamed side long, whether they run beside each other or in turn), a little more where the streamed side is read more often,
 // a little less at 32 columns, where several workgroups of one wavefront's tiles fit a compute unit. Forward / dQ / dK and dV, us,
-// one against two wavefronts of rows where both leave two units of work: 45 x 171 x 6 chunks at 32 34 / 45 / - and 39 / 50 / -, 16 x 700 x 4 at
-// 64 126 / 208 and 141 / 183, 24 x 350 x 5 at 80 178 / 223 and 119 / 157, 12 x 800 x 3 at 96 302 / 364 and 165 / 219. Whole steps before (a
-// launch a chunk of 128 rows each, 80 and 96 columns as 128 with copies) and now: 322 -> 121, 1061 -> 490, 1707 -> 435, 1960 -> 576;
-// launches that filled the chip 1963 -> 1875 (64 x 1000 x 3 at 64: 0.09 PFLOP/s of the matrix cores' 0.16) and 5410 -> 4860 (48 x 900 x 4 at 128).
+// one against two wavefronts of rows where both leave two units of work, each summed in one chain: 45 x 171 x 6 chunks at 32 34 / 45 / - and
+// 39 / 50 / -, 16 x 700 x 4 at 64 126 / 208 and 141 / 183, 12 x 800 x 3 at 96 302 / 364 and 165 / 219. Whole steps before (a launch a chunk of
+// 128 rows each, 96 columns as 128 with copies) and now: 322 -> 122, 1061 -> 501, 1960 -> 594; a launch that filled the chip 1963 -> 1892
+// (64 x 1000 x 3 at 64: 0.09 PFLOP/s of the matrix cores' 0.16).
 int width(long long rows, long long entries, int d, int least) {
   int best = 4;
   long long best_cost = -1;

@@ -1757,7 +1757,7 @@ Tiling tiling_of(const Launch& L, int Hout, int Wout, bool wide_rows, bool even,
   // of their t + 1 tile columns and u + 1 rows cost as much as a whole one (staged rows, barriers) for what little they hold.
   // Rows of x then start at the first staged column, on cache lines where they are whole lines themselves. Gradient with the fold
   // of 2 x 32 -> 32 channels of 128^3 429 -> 338 us (16 tiles a plane for 27), at stride 2 of 4 x 64 -> 128 of 256 x 256 53.5 -> 34.8 (one
-  // tile a workgroup for two), 4 x 32 -> 32 of 256 x 256 26.3 -> 21.6, 8 x 8 -> 24 of 64 x 512 24.9 -> 20.2.
+  // tile a workgroup for two).
   auto spare = [](int extent, int pad, int tile) {
     return (pad == 1 || pad == 2) && extent > pad && (extent - pad + tile - 1) / tile < (extent + tile - 1) / tile ? pad : 0;
   };
@@ -1769,10 +1769,9 @@ Tiling tiling_of(const Launch& L, int Hout, int Wout, bool wide_rows, bool even,
   };
   // 64 produced channels a tile where they pad no further than 32 and the tiles go round: a tile of 32 takes 0.55 to 0.65 of the time of
   // one of 64 (the same rows staged, half of the products; 0.8 in the strided forward, whose tiles hold fewer), and where the chip is not
-  // full twice as many of them run beside each other. Forward of 2 x 64 -> 64 of 128 x 128 24.2 -> 17.0 us, 1 x 64 -> 64 of 256 x 256
-  // 24.9 -> 18.2, 2 x 128 -> 128 of 128 x 128 39 -> 27, 1 x 70 -> 55 of 69 x 38 32 -> 21; gradient with the fold of 4 x 64 -> 64 of 256 x 256
-  // (512 tiles of 32 with the rows and columns beside them for 340 of 64) 50 -> 42. Forced, where the chip is full: 4 x 64 -> 64 of
-  // 256 x 256 forward 30.5 -> 33.2, 5 x 49 -> 59 of 586 x 314 105 -> 120. Tiles at the edge take about a tenth longer for rows above them.
+  // full twice as many of them run beside each other. Forward of 2 x 64 -> 64 of 128 x 128 24.2 -> 17.0 us, gradient with the fold of
+  // 4 x 64 -> 64 of 256 x 256 (512 tiles of 32 with the rows and columns beside them for 340 of 64) 50 -> 42; forced, where the chip is
+  // full, 5 x 49 -> 59 of 586 x 314 forward 105 -> 120. Tiles at the edge take about a tenth longer for rows above them.
   Tiling best{};
   double least = 0.0;
   for (const int MT : {64, 32}) {

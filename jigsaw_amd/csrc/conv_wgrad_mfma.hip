@@ -101,7 +101,7 @@ struct WgradParams {
 // volume have two parts, the halves of the columns; a 6-wavefront shape gets two more wavefronts that only help with the prefetch.
 // Blocks with one or two pairs have four, at stride 1 the quarters of the columns, at stride 2 halves of each row: with two
 // parts there was one wavefront a SIMD, and what it did between its matrix instructions (loads, moves to LDS, the barrier)
-// nothing ran beside; a part's fewer fragments leave room for two (200 to 240 registers, 300 to 320 before).
+// nothing ran beside; a part's fewer fragments leave room for two (200 to 256 registers; 302 to 320 before, 400 to 435 at stride 2).
 // Partials and their reduction included: 2 x 40 -> 72 of 217 x 301 bf16 51 -> 44 us, 4 x 32 -> 64 of 512 x 512 80 -> 73, 7 x 5 -> 118
 // of 229 x 380 92 -> 83, at stride 2 of 6 x 91 -> 23 of 244 x 446 76 -> 64 and of 2 x 77 -> 211 of 436 x 84 80 -> 57; the smallest
 // layers (2 x 20 -> 33 of 100 x 150, 23 us) wait for the setup, the partials and the second launch, as before.
