@@ -23,8 +23,11 @@
 //   Workgroup: 8 wavefronts (dQ: 4 in small launches; dK/dV: 4) = 4 or 2 blocks of 32 rows (queries
 //   for dQ, keys for dK/dV) x 2 halves of the streamed side, combined through LDS.
 //   Streamed tiles (64 rows x 128 bytes; 32 rows where dQ has 2 blocks) travel from memory straight into LDS, row-major
-//   with the 16-byte chunks of a row XOR-swizzled by row % 8 (no registers, no vector
-//   instructions, no second, transposed copy): the transposed fragments come from
+//   with the 16-byte chunks of a row XOR-swizzled by row / 2 % 8 (no registers, no vector
+//   instructions, no second, transposed copy). LDS has 64 banks, two of these rows, so that the 16 rows a
+//   row fragment's read takes at a time meet all of them once; with row % 8 rows r and r + 8 lay on the same
+//   ones (reads of eight wavefronts 294 : 460 bytes per ns and compute unit, transposed reads 300 either way; traced, 8 heads x
+//   4096 x 4 chunks: dQ 222 -> 213 us, dK/dV 327 -> 310). The transposed fragments come from
 //   ds_read_b64_tr_b16 (within 16 lanes, lane i receives element i % 4 of the 8 bytes
 //   that lanes i / 4 + 4 j point at, j = 0..3), two reads of 4 consecutive rows each.
 //
@@ -73,35 +76,36 @@ __device__ __forceinline__ bf16x8 lds_frag(const unsigned char* p) {
 }
 
 // Offsets of a lane in a transfer of 8 rows (jg::to_lds_1k): lane L sits at row L / 8, chunk position L % 8 and
-// fetches chunk (L % 8) ^ (row % 8) of its row. First for rows first_row + 0..7 of a tensor of `rows` rows, clamped to its last one.
-__device__ __forceinline__ uint32_t dma_clamped_offset(int lane, int first_row, int rows) {
-  return (uint32_t)min(first_row + (lane >> 3), rows - 1) * ROWB + (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4);
+// fetches chunk (L % 8) ^ (row / 2 % 8) of its row; `second`: rows 8 .. 15 of 16. First for rows first_row + 0..7 of a tensor of
+// `rows` rows, clamped to its last one.
+__device__ __forceinline__ uint32_t dma_clamped_offset(int lane, int first_row, int rows, int second) {
+  return (uint32_t)min(first_row + (lane >> 3), rows - 1) * ROWB + (uint32_t)(((lane & 7) ^ (lane >> 4) ^ (4 * second)) << 4);
 }
 __device__ __forceinline__ uint32_t dma_lane_offset(int lane) {
-  return (uint32_t)((lane >> 3) * ROWB + (((lane & 7) ^ (lane >> 3)) << 4));
+  return (uint32_t)((lane >> 3) * ROWB + (((lane & 7) ^ (lane >> 4)) << 4));  // the second 8 rows of 16: ^ 64
 }
 
 // fragment of a row-major tile: row r (0..63), 16-byte chunk c (0..7)
 __device__ __forceinline__ bf16x8 nat_frag(const unsigned char* nat, int r, int c) {
-  return lds_frag(nat + r * ROWB + ((c ^ (r & 7)) << 4));
+  return lds_frag(nat + r * ROWB + ((c ^ ((r >> 1) & 7)) << 4));
 }
 
 // Per-lane constant part of the address of a TRANSPOSED fragment (A operand: 32 columns of the
 // tile x 16 of its rows): lane p of a group of 16 points at row +4 kg + p / 4, columns 32 nb +
-// 16 (group % 2) + 4 (p % 4); the row's swizzle is 4 kg + p / 4 whatever multiple of 8 the
-// fragment starts at.
+// 16 (group % 2) + 4 (p % 4); the row's swizzle is (4 kg + p / 4) / 2 whatever multiple of 16 the
+// fragment starts at, and 4 more eight rows further on: the place of the other block there.
 __device__ __forceinline__ int tr_lane_offset(int lane, int nb) {
   const int pp = lane & 15, g1 = (lane >> 4) & 1, kg = lane >> 5;
-  const int rsw = 4 * kg + (pp >> 2);
-  return rsw * ROWB + (((4 * nb + 2 * g1 + ((pp & 3) >> 1)) ^ rsw) << 4) + 8 * (pp & 1);
+  const int row = 4 * kg + (pp >> 2);
+  return row * ROWB + (((4 * nb + 2 * g1 + ((pp & 3) >> 1)) ^ (row >> 1)) << 4) + 8 * (pp & 1);
 }
 // Transposed fragment whose 16 rows start at `row0` (a multiple of 16): slots 0..3 = rows
 // row0 + 4 kg + 0..3, slots 4..7 = rows row0 + 8 + 4 kg + 0..3: the order an accumulator lane
 // holds its rows in.
-__device__ __forceinline__ bf16x8 tr_frag(const unsigned char* nat, int lane_off, int row0) {
+__device__ __forceinline__ bf16x8 tr_frag(const unsigned char* nat, const int (&lane_off)[2], int nb, int row0) {
   typedef __attribute__((address_space(3))) i16x4* tr_ptr;
-  const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(nat + lane_off + row0 * ROWB));
-  const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(nat + lane_off + (row0 + 8) * ROWB));
+  const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(nat + lane_off[nb] + row0 * ROWB));
+  const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(nat + lane_off[nb ^ 1] + (row0 + 8) * ROWB));
   u32x4 w;
   w.x = __builtin_bit_cast(u32x2, lo).x;
   w.y = __builtin_bit_cast(u32x2, lo).y;
@@ -189,14 +193,14 @@ __global__ __launch_bounds__(DqPlan<QB>::THREADS, QB == 2 ? 2 : 1) void attn_bwd
   // row fragments: row ln of a 32-row block, chunk 2 c + kg
   int row_off[4];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) row_off[c] = ln * ROWB + (((2 * c + kg) ^ (ln & 7)) << 4);
+  for (int c = 0; c < 4; ++c) row_off[c] = ln * ROWB + (((2 * c + kg) ^ ((ln >> 1) & 7)) << 4);
 
   // K and V of tile t straight into its buffer (free since the barrier that ended the tile before)
   auto issue_loads = [&](int slot) {  // called with slot = 0, 1, 2, 3, 0, ... in turn
     const uint32_t dst = lds_dma + (uint32_t)(slot * DQ_BUF);
     const int row = row_first + ld_tile * DQ_BT;
     if (RAGGED) {
-      const uint32_t o0 = dma_clamped_offset(lane, row, p.sk), o1 = dma_clamped_offset(lane, row + 8, p.sk);
+      const uint32_t o0 = dma_clamped_offset(lane, row, p.sk, 0), o1 = dma_clamped_offset(lane, row + 8, p.sk, 1);
       jg::to_lds_1k(kdma, o0, dst);
       jg::to_lds_1k(kdma, o1, dst + 8 * ROWB);
       jg::to_lds_1k(vdma, o0, dst + DQ_NAT);
@@ -204,9 +208,9 @@ __global__ __launch_bounds__(DqPlan<QB>::THREADS, QB == 2 ? 2 : 1) void attn_bwd
     } else {
       const long long off = (long long)row * ROWB;
       jg::to_lds_1k(kdma + off, dma_off, dst);
-      jg::to_lds_1k(kdma + off + 8 * ROWB, dma_off, dst + 8 * ROWB);
+      jg::to_lds_1k(kdma + off + 8 * ROWB, dma_off ^ 64u, dst + 8 * ROWB);
       jg::to_lds_1k(vdma + off, dma_off, dst + DQ_NAT);
-      jg::to_lds_1k(vdma + off + 8 * ROWB, dma_off, dst + DQ_NAT + 8 * ROWB);
+      jg::to_lds_1k(vdma + off + 8 * ROWB, dma_off ^ 64u, dst + DQ_NAT + 8 * ROWB);
     }
     if (++ld_tile == tiles_per_chunk && ld_chunk + 1 < p.nchunks) {
       ld_tile = 0;
@@ -281,7 +285,7 @@ __global__ __launch_bounds__(DqPlan<QB>::THREADS, QB == 2 ? 2 : 1) void attn_bwd
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb)
-        dq[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(kn, tr_off[nb], sb * 32 + 16 * t), ds_prev[t], dq[nb], 0, 0, 0);
+        dq[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(kn, tr_off, nb, sb * 32 + 16 * t), ds_prev[t], dq[nb], 0, 0, 0);
   };
   // one step of the pipeline: A of (k_next, sb_next), B of the current block, C of (k_prev, sb_prev)
   int keys_left = p.sk - ks_u * tiles_per_chunk * DQ_BT, tile_at = 0;  // RAGGED: keys from the current block's first one on
@@ -431,7 +435,7 @@ __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void at
     for (int r = 0; r < DKV_SHARE; r += 8) {
       const int row = row_first + t * BT + r;
       const long long off = RAGGED ? 0 : (long long)row * ROWB;
-      const uint32_t lane_off = RAGGED ? dma_clamped_offset(lane, row, p.sq) : dma_off;
+      const uint32_t lane_off = RAGGED ? dma_clamped_offset(lane, row, p.sq, r >> 3 & 1) : dma_off ^ (8u * (uint32_t)(r & 8));
       jg::to_lds_1k(qdma + off, lane_off, dst + r * ROWB);
       jg::to_lds_1k(ddma + off, lane_off, dst + NAT + r * ROWB);
     }
@@ -523,8 +527,8 @@ __global__ __launch_bounds__(DKV_THREADS, 8 / (2 * DKV_KB) >= 2 ? 2 : 1) void at
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) {
-          dv[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(dn, tr_off[nb], sb * 32 + 16 * t), pf[sb][t], dv[nb], 0, 0, 0);
-          dk[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(qn, tr_off[nb], sb * 32 + 16 * t), dsf[sb][t], dk[nb], 0, 0, 0);
+          dv[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(dn, tr_off, nb, sb * 32 + 16 * t), pf[sb][t], dv[nb], 0, 0, 0);
+          dk[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(qn, tr_off, nb, sb * 32 + 16 * t), dsf[sb][t], dk[nb], 0, 0, 0);
         }
   };
 

@@ -17,7 +17,7 @@
 //   Tiles            K and V tiles (32 keys x 128 bytes) travel from memory straight into
 //                    LDS (global_load_lds, 16 bytes per lane, no registers, no vector
 //                    instructions); the 16-byte chunks of a row are XOR-swizzled with
-//                    row % 8 by choosing which chunk a lane fetches. Four buffers per key
+//                    row / 2 % 8 by choosing which chunk a lane fetches (why: attn_bwd_mfma.hip). Four buffers per key
 //                    quarter, filled three tiles ahead. The fragment addresses are per-lane
 //                    constants: the loop spends its vector instructions on the softmax.
 //   Operand reuse    every MFMA takes one fragment from LDS (1 KB per wavefront), so a
@@ -149,13 +149,13 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
 
   // ---- tiles: memory -> LDS directly. One instruction of a wavefront lands 64 x 16 bytes
   // contiguously in lane order = 8 rows; lane L sits at row L / 8, chunk position L % 8 and
-  // fetches the chunk (L % 8) ^ (row % 8) of its row. A wavefront moves rows 16 qg .. 16 qg + 15
+  // fetches the chunk (L % 8) ^ (row / 2 % 8) of its row. A wavefront moves rows 16 qg .. 16 qg + 15
   // of the K tile and of the V tile (two instructions each).
   // The base is wave-uniform (tile and row block, advanced with scalar arithmetic) and the lane's offset constant, so that
   // issuing a tile costs no vector instruction (jg::to_lds_1k). A buffer is read only after the wait + barrier that
   // follows its transfer, and refilled only after the barrier that follows its last read.
-  const uint32_t dma_swz = (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4);
-  const uint32_t dma_off = (uint32_t)((lane >> 3) * ROWB) + dma_swz;
+  const uint32_t dma_swz = (uint32_t)(((lane & 7) ^ (lane >> 4)) << 4);  // of rows 0 .. 7 of 16; the other eight: ^ 64
+  const uint32_t dma_off = (uint32_t)((lane >> 3) * ROWB) + dma_swz, dma_off8 = dma_off ^ 64u;
   const int qg_u = __builtin_amdgcn_readfirstlane(qg), kq_u = __builtin_amdgcn_readfirstlane(kq);
   const uint32_t lds_dma = jg::lds_address(smem) + (uint32_t)(kq_u * QUARTER_BYTES + 16 * qg_u * ROWB);
   // the load cursor: tiles are requested in stream order, the last one again and again past the end
@@ -168,9 +168,9 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
     const uint32_t dst = lds_dma + (uint32_t)(buf * TILE_BYTES);
     const long long off = (long long)(row_first + ld_tile * BN) * ROWB;
     jg::to_lds_1k(kdma + off, dma_off, dst);
-    jg::to_lds_1k(kdma + off + 8 * ROWB, dma_off, dst + 8 * ROWB);
+    jg::to_lds_1k(kdma + off + 8 * ROWB, dma_off8, dst + 8 * ROWB);
     jg::to_lds_1k(vdma + off, dma_off, dst + KV_BYTES);
-    jg::to_lds_1k(vdma + off + 8 * ROWB, dma_off, dst + KV_BYTES + 8 * ROWB);
+    jg::to_lds_1k(vdma + off + 8 * ROWB, dma_off8, dst + KV_BYTES + 8 * ROWB);
     if (ld_left > 0) {
       --ld_left;
       if (++ld_tile == qtiles) {
@@ -182,20 +182,21 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
     }
   };
   // per-lane constant parts of the fragment addresses
-  //   K fragment c of key row ln: logical chunk 2 c + kg, stored at chunk (2 c + kg) ^ (ln % 8)
+  //   K fragment c of key row ln: logical chunk 2 c + kg, stored at chunk (2 c + kg) ^ (ln / 2 % 8)
   int kaddr[4];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) kaddr[c] = ln * ROWB + (((2 * c + kg) ^ (ln & 7)) << 4);
+  for (int c = 0; c < 4; ++c) kaddr[c] = ln * ROWB + (((2 * c + kg) ^ ((ln >> 1) & 7)) << 4);
   //   V^T fragment (dv block nb, K-step tt) = two transpose reads (r = 0, 1) of the 4 keys
   //   16 tt + 8 r + 4 kg + 0..3: lane p of a group of 16 points at key row +p / 4, dv 32 nb +
-  //   16 (group % 2) + 4 (p % 4); the row's swizzle is (4 kg + p / 4), the same for every (tt, r)
+  //   16 (group % 2) + 4 (p % 4); the row's swizzle is 4 r + (4 kg + p / 4) / 2, so that the second read of a block is
+  //   the first one of the other block eight rows further on
   int vaddr[2];
   {
     const int pp = lane & 15, g1 = (lane >> 4) & 1;
-    const int rsw = 4 * kg + (pp >> 2);
+    const int row = 4 * kg + (pp >> 2);
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb)
-      vaddr[nb] = rsw * ROWB + (((4 * nb + 2 * g1 + ((pp & 3) >> 1)) ^ rsw) << 4) + 8 * (pp & 1);
+      vaddr[nb] = row * ROWB + (((4 * nb + 2 * g1 + ((pp & 3) >> 1)) ^ (row >> 1)) << 4) + 8 * (pp & 1);
   }
 
   f32x16 o[2][2];  // [query block][dv block] O^T: lane = query, register i = dv nb*32 + 8*(i/4) + 4*kg + i%4
@@ -226,7 +227,7 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
       for (int tt = 0; tt < 2; ++tt) {
         typedef __attribute__((address_space(3))) i16x4* tr_ptr;
         const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(vt + vaddr[nb] + (16 * tt) * ROWB));
-        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(vt + vaddr[nb] + (16 * tt + 8) * ROWB));
+        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(vt + vaddr[nb ^ 1] + (16 * tt + 8) * ROWB));
         u32x4 w;
         w.x = __builtin_bit_cast(u32x2, lo).x;
         w.y = __builtin_bit_cast(u32x2, lo).y;
@@ -387,7 +388,7 @@ __global__ __launch_bounds__(THREADS) void attn_fwd_mfma_kernel(ChunkTable, FwdA
     const int valid = tail - kq_u * BN;  // keys of this quarter's tile, <= 0: none
     const int row = qtiles * NQ * BN + kq_u * BN + 16 * qg_u;
     const uint32_t o0 = (uint32_t)min(row + (lane >> 3), p.sk - 1) * ROWB + dma_swz;
-    const uint32_t o1 = (uint32_t)min(row + 8 + (lane >> 3), p.sk - 1) * ROWB + dma_swz;
+    const uint32_t o1 = (uint32_t)min(row + 8 + (lane >> 3), p.sk - 1) * ROWB + (dma_swz ^ 64u);
     auto dma_tail = [&](int chunk, int buf) {
       const uint32_t dst = lds_dma + (uint32_t)(buf * TILE_BYTES);
       const char* kc = chunk_entry(0, chunk) + chunk_off;
