@@ -18,10 +18,11 @@
 //   proj_tn_kernel   part[split](n, c) = sum_{r in split} g(r, n) * x(r, c)   (weight gradient;
 //                    bias gradient sum_r g(r, n) on the way), then proj_reduce_kernel
 //
-// bf16 on v_mfma_f32_32x32x16_bf16 with fp32 accumulation. Workgroup tiles of 256 x 256 (eight wavefronts
-// of 128 x 64), 128 x 128 and, NT, 64 x 64 (four wavefronts); the operands travel from memory straight
-// into LDS, 64 contraction elements a stage, one stage ahead of the MFMAs.
+// bf16 on v_mfma_f32_32x32x16_bf16 with fp32 accumulation. Workgroup tiles of 256 x 256 and 128 x 128 (eight wavefronts)
+// and, NT, 64 x 64 (four); the operands travel from memory straight into LDS, 64 contraction elements a stage, one
+// stage ahead of the MFMAs.
 // proj_generic_kernel covers the other dtypes and unaligned shapes with plain FMAs.
+#include <algorithm>
 #include <type_traits>
 
 #include "lds_transfer.h"
@@ -37,10 +38,25 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
+// Division by a number that holds for a whole launch, of numbers below 2^31: m = 2^(32 + s) / d rounded up, s < 0 for d = 1. A division of
+// the compiler's own is 30 instructions and more, over 100 in 64 bits, and the offsets of a tile take a dozen (see proj_nt_kernel).
+struct Div {
+  uint32_t m;
+  int s;
+};
+Div div_by(int d) {
+  if (d <= 1) return {0u, -1};
+  int bits = 0;
+  while ((1ll << bits) < d) ++bits;
+  return {(uint32_t)(((1ull << (31 + bits)) + d - 1) / d), bits - 1};
+}
+__device__ __forceinline__ uint32_t quotient(uint32_t n, const Div& d) { return d.s < 0 ? n : __umulhi(n, d.m) >> d.s; }
+
 struct Map {
   int heads;     // 0: row-major with leading dimension ld; 1: (t, B, H, S, D)
   long long ld;
   int B, H, S, D;
+  Div by_S, by_D, by_H;
 };
 
 __device__ __forceinline__ long long row_part(const Map& m, long long r) {
@@ -55,28 +71,47 @@ __device__ __forceinline__ long long feat_part(const Map& m, int j) {
   return ((long long)t * m.B * m.H + h) * m.S * m.D + d;
 }
 
-// Walks consecutive tokens without a division per token.
-struct RowWalk {
-  long long b, s;  // heads: batch entry and position; row-major: s = token
+// The same as byte offsets, of tokens and features below 2^31. OFF: uint32_t where the tensor has fewer than 2^32 bytes.
+template <typename OFF>
+__device__ __forceinline__ OFF row_bytes(const Map& m, uint32_t r) {
+  if (!m.heads) return (OFF)r * (OFF)m.ld * 2u;
+  const uint32_t b = quotient(r, m.by_S), s = r - b * (uint32_t)m.S;
+  return ((OFF)b * (OFF)m.H * (OFF)m.S + s) * (OFF)m.D * 2u;
+}
+template <typename OFF>
+__device__ __forceinline__ OFF feat_bytes(const Map& m, uint32_t j) {
+  if (!m.heads) return (OFF)j * 2u;
+  const uint32_t hd = quotient(j, m.by_D), t = quotient(hd, m.by_H), d = j - hd * (uint32_t)m.D, h = hd - t * (uint32_t)m.H;
+  return (((OFF)t * (OFF)m.B * (OFF)m.H + h) * (OFF)m.S * (OFF)m.D + d) * 2u;
+}
+
+// Tokens r, r + step, ... of a tensor as byte offsets; heads: (b * H * S + s) * D, row-major: r * ld.
+template <typename OFF>
+struct TokenWalk {
+  OFF off;         // bytes
+  int s, S;        // position in the batch entry and its length
+  OFF row, jump;   // bytes between tokens of an entry; extra bytes from the end of an entry to the next one
   __device__ __forceinline__ void start(const Map& m, long long r) {
-    if (m.heads) {
-      b = r / m.S;
-      s = r - b * m.S;
-    } else {
-      b = 0;
-      s = r;
-    }
+    row = (OFF)(m.heads ? m.D : m.ld) * 2u;
+    S = m.heads ? m.S : 0x7fffffff;
+    jump = m.heads ? (OFF)(m.H - 1) * (OFF)m.S * row : 0u;
+    const long long b = !m.heads ? 0 : r < (1ll << 31) ? (long long)quotient((uint32_t)r, m.by_S) : r / m.S;
+    s = m.heads ? (int)(r - b * m.S) : 0;
+    off = m.heads ? ((OFF)b * (OFF)m.H * (OFF)m.S + (OFF)s) * row : (OFF)r * row;
   }
-  __device__ __forceinline__ void advance(const Map& m, int by) {
+  __device__ __forceinline__ void advance(int by) {
     s += by;
-    if (m.heads)
-      while (s >= m.S) {
-        s -= m.S;
-        ++b;
+    off += (OFF)by * row;
+    if (S >= by) {  // wave-uniform: one entry further at most
+      const bool over = s >= S;
+      s -= over ? S : 0;
+      off += over ? jump : (OFF)0;
+    } else {
+      while (s >= S) {
+        s -= S;
+        off += jump;
       }
-  }
-  __device__ __forceinline__ long long part(const Map& m) const {
-    return m.heads ? (b * m.H * m.S + s) * m.D : s * m.ld;
+    }
   }
 };
 
@@ -93,6 +128,7 @@ struct NtParams {
   long long rows;
   int N, K;
   int tiles_n, tiles;
+  Div by_tiles_n;
   // What happens to a result on its way out (the values are the bf16-rounded acc + bias, as a
   // separate elementwise pass over the stored tensor would see them; arithmetic in fp32):
   //   EPI_NONE  out = y
@@ -154,21 +190,25 @@ template <int IM, int JN, int WM, int WN>
 struct NtShape {
   static constexpr int TM = 32 * IM * WM, TNF = 32 * JN * WN;  // tokens, features of a tile
   static constexpr int WAVES = WM * WN, THREADS = 64 * WAVES;
-  static constexpr int ROWB = BK * 2;                          // bytes of a row of a stage: 8 chunks of 8 k, chunk c at c ^ (row % 8)
+  static constexpr int ROWB = BK * 2;                          // bytes of a row of a stage: 8 chunks of 8 k, chunk c at c ^ (row / 2 % 8)
   static constexpr int OP_A = TM * ROWB, OP_W = TNF * ROWB, STAGE = OP_A + OP_W;
   static constexpr int LDS = 2 * STAGE + 2 * TNF * 4;          // two stages, then the bias of two tiles as floats
   static constexpr int DMA_A = TM / 8 / WAVES, DMA_W = TNF / 8 / WAVES;  // 1 KB transfers (8 rows) of a wavefront per stage
   static constexpr int OUT_PITCH = 32 * JN * 2 + 16;           // bytes per token of a wavefront's block in LDS
   static_assert(TM % (8 * WAVES) == 0 && TNF % (8 * WAVES) == 0, "whole transfers");
+  static_assert(WAVES % 2 == 0, "a wavefront's transfers start at the same row % 16");
   static_assert(32 * OUT_PITCH * WAVES <= STAGE, "the results pass through the stage just computed");
 };
 
 // Persistent workgroups walk the tiles of one XCD's contiguous range (consecutive tiles share a panel of `a`, which
 // meets in one L2). The transfers of a stage are issued a stage ahead, across tile borders too, so that the first
 // stage of a tile arrives under the last one of the tile before and under its epilogue: with K = 512 a tile is only
-// eight stages long. Bound by the matrix cores and, beside them, by the LDS reads (3/4 KB per matrix instruction in
-// the 256 x 256 tile). 32768 tokens: 512 -> 1536 features 57.6 us (894 TFLOP/s; staged through registers, a tile per
-// workgroup: 68.1), 1536 -> 512 53.2 us (59.5), 512 -> 512 23.8 us (26.2); 65536 tokens, 128 -> 384 19.1 us (23.2).
+// eight stages long. A stage of the 256 x 256 tile is 2048 cycles of matrix instructions and takes 3300: the rest are the barrier, where
+// wavefronts wait 550 for the last one, and what precedes the first matrix instruction behind it. What the vector unit does there and between
+// tiles counts in full: offsets by the compiler's divisions were 0.7 to 1.1 us a tile (0.35 by Div), the epilogue's by 64-bit products 1.3
+// (0.8). The 128 x 128 tile as eight wavefronts of 64 x 32 has two to a SIMD and, with a second workgroup, four (four of 64 x 64
+// before: 0.75 us a stage, 0.55 now). us before -> now: 32768 tokens, 512 -> 1536 features 59.7 -> 57.6 (894 TFLOP/s), 1536 -> 512 52.7 -> 49.5,
+// 512 -> 512 24.0 -> 22.7; 65536, 128 -> 384 19.4 -> 17.5; 2680, 896 -> 896 15.5 -> 12.2, 468, 2112 -> 704 17.1 -> 14.8.
 template <int IM, int JN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_nt_kernel(NtParams p) {
   typedef NtShape<IM, JN, WM, WN> SH;
@@ -189,8 +229,8 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_nt_ke
   auto tile_at = [&](int i) { return t_begin + slot + i * wg_per_xcd; };
 
   // ---- load cursor. Lane L of a transfer sits at row L / 8, chunk position L % 8, and fetches chunk
-  // (L % 8) ^ (row % 8), the same one in every transfer.
-  const int chunk = (lane & 7) ^ (lane >> 3);
+  // (L % 8) ^ (row / 2 % 8), the same one in every transfer (they are 16 rows or a multiple of it apart).
+  const int chunk = (lane & 7) ^ ((wave & 1) << 2 | lane >> 4);
   uint32_t a_row[SH::DMA_A], w_row[SH::DMA_W];
   int ld_tile = -1, ld_ks = 0;
   uint16_t bias_next = 0;  // raw: converted when it goes to LDS, a use here would wait for the load
@@ -198,31 +238,35 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_nt_ke
   auto enter_tile = [&]() {
     ++ld_tile;
     ld_ks = 0;
-    const int t = tile_at(ld_tile);
-    const long long m0 = (long long)(t / p.tiles_n) * TM;
-    const int n0 = (t % p.tiles_n) * TNF;
+    const uint32_t t = tile_at(ld_tile), tm = quotient(t, p.by_tiles_n);
+    const int n0 = (t - tm * p.tiles_n) * TNF;
 #pragma unroll
-    for (int i = 0; i < SH::DMA_A; ++i) {
-      long long r = m0 + (i * SH::WAVES + wave) * 8 + (lane >> 3);
-      if (r > p.rows - 1) r = p.rows - 1;  // a row past the end repeats the last one and is dropped
-      a_row[i] = (uint32_t)(row_part(p.am, r) * 2);
-    }
+    for (int i = 0; i < SH::DMA_A; ++i)  // a row past the end repeats the last one and is dropped
+      a_row[i] = row_bytes<uint32_t>(p.am, min(tm * TM + (i * SH::WAVES + wave) * 8 + (lane >> 3), (uint32_t)p.rows - 1));
 #pragma unroll
     for (int i = 0; i < SH::DMA_W; ++i) {
       const int n = min(n0 + (i * SH::WAVES + wave) * 8 + (lane >> 3), p.N - 1);
-      w_row[i] = (uint32_t)((long long)n * p.K * 2);
+      w_row[i] = (uint32_t)n * (uint32_t)p.K * 2u;
     }
     if (p.bias != nullptr) bias_next = p.bias[min(n0 + tid, p.N - 1)];  // features past the end are dropped
   };
   const uint32_t lds_a = jg::lds_address(smem) + wave_u * 1024, lds_w = lds_a + SH::OP_A;
-  auto issue = [&](int buf) {
+  uint32_t fa = 0, fw = 0;  // where the stage to fetch lies in a row
+  auto enter_stage = [&]() {
     const int k = ld_ks * BK + chunk * 8;
     const int kk = k < p.K ? k : 0;  // a chunk past the contraction length is read at k = 0 and zeroed below
-    const uint32_t fa = (uint32_t)(feat_part(p.am, kk) * 2), fw = (uint32_t)kk * 2;
+    fa = feat_bytes<uint32_t>(p.am, kk);
+    fw = (uint32_t)kk * 2u;
+  };
+  constexpr int TRANSFERS = SH::DMA_A + SH::DMA_W;
+  auto transfer = [&](int q, int buf) __attribute__((always_inline)) {
+    if (q < SH::DMA_A) jg::to_lds_1k(p.a, a_row[q] + fa, lds_a + buf * SH::STAGE + q * SH::WAVES * 1024);
+    else jg::to_lds_1k(p.w, w_row[q - SH::DMA_A] + fw, lds_w + buf * SH::STAGE + (q - SH::DMA_A) * SH::WAVES * 1024);
+  };
+  auto issue = [&](int buf) {
+    enter_stage();
 #pragma unroll
-    for (int i = 0; i < SH::DMA_A; ++i) jg::to_lds_1k(p.a, a_row[i] + fa, lds_a + buf * SH::STAGE + i * SH::WAVES * 1024);
-#pragma unroll
-    for (int i = 0; i < SH::DMA_W; ++i) jg::to_lds_1k(p.w, w_row[i] + fw, lds_w + buf * SH::STAGE + i * SH::WAVES * 1024);
+    for (int q = 0; q < TRANSFERS; ++q) transfer(q, buf);
   };
   // the last stage of a contraction length that is no multiple of BK: a lane clears what its transfers put past it
   auto clear_tail = [&](int buf, int ks) {
@@ -235,29 +279,43 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_nt_ke
 
   f32x16 acc[IM][JN];
   // acc[i][j] = w fragment (rows: features) x a fragment (columns: tokens). The fragments of
-  // the next 16-wide step are requested before the MFMAs of this one are issued.
-  auto compute = [&](int buf) {
+  // a 16-wide step are requested AHEAD steps before its MFMAs are issued.
+  constexpr int AHEAD = IM * JN == 1 ? BK / 16 : IM * JN <= 4 ? 2 : 1;
+  constexpr bool SPREAD = IM * JN > 1;
+  constexpr int EVERY = IM * JN >= 8 ? 2 : 1;
+  static_assert(EVERY * TRANSFERS <= BK / 16 * IM * JN, "every transfer has its place");
+  // The transfers of a stage to come (buffer `to`, none: -1) go out one by one between them: eight wavefronts' 64 at the head of
+  // a stage occupied the address unit for 1000 cycles in which no matrix instruction was issued.
+  auto compute = [&](int buf, int to) {
     const unsigned char* sa = smem + buf * SH::STAGE + (wm * 32 * IM + ln) * ROWB;
     const unsigned char* sw = smem + buf * SH::STAGE + SH::OP_A + (wn * 32 * JN + ln) * ROWB;
-    u32x4 fr[2][IM + JN];
+    u32x4 fr[AHEAD + 1][IM + JN];
     auto fetch = [&](int kk, u32x4 (&f)[IM + JN]) {
-      const int at = ((kk * 2 + kg) ^ (ln & 7)) << 4;
+      const int at = ((kk * 2 + kg) ^ ((ln >> 1) & 7)) << 4;
 #pragma unroll
       for (int t = 0; t < IM; ++t) f[t] = *reinterpret_cast<const u32x4*>(sa + t * 32 * ROWB + at);
 #pragma unroll
       for (int t = 0; t < JN; ++t) f[IM + t] = *reinterpret_cast<const u32x4*>(sw + t * 32 * ROWB + at);
     };
-    fetch(0, fr[0]);
+#pragma unroll
+    for (int kk = 0; kk < AHEAD; ++kk) fetch(kk, fr[kk]);
 #pragma unroll
     for (int kk = 0; kk < BK / 16; ++kk) {
-      if (kk + 1 < BK / 16) fetch(kk + 1, fr[(kk + 1) & 1]);
+      if (kk + AHEAD < BK / 16) fetch(kk + AHEAD, fr[(kk + AHEAD) % (AHEAD + 1)]);
+      const u32x4(&f)[IM + JN] = fr[kk % (AHEAD + 1)];
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < IM; ++i)
 #pragma unroll
-        for (int j = 0; j < JN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fr[kk & 1][IM + j]),
-                                                              __builtin_bit_cast(bf16x8, fr[kk & 1][i]), acc[i][j], 0, 0, 0);
+        for (int j = 0; j < JN; ++j) {
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, f[IM + j]), __builtin_bit_cast(bf16x8, f[i]), acc[i][j], 0, 0, 0);
+          const int at = (kk * IM + i) * JN + j;
+          if (SPREAD && at % EVERY == EVERY - 1 && at / EVERY < TRANSFERS) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (to >= 0) transfer(at / EVERY, to);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -286,19 +344,21 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_nt_ke
     unsigned char* block = smem + buf * SH::STAGE + wave * 32 * SH::OUT_PITCH;
     constexpr int CPR = JN * 4, RPI = 64 / CPR;  // pieces per token, tokens per store instruction
     const int fc = lane % CPR, trow = lane / CPR;
-    const int n = (t % p.tiles_n) * TNF + wn * 32 * JN + fc * 8;
-    const long long r0 = (long long)(t / p.tiles_n) * TM + wm * 32 * IM + trow;
-    const long long fo = feat_part(p.om, n < p.N ? n : 0);
-    RowWalk rwk, ahead;
-    rwk.start(p.om, r0);
-    ahead = rwk;
+    const uint32_t tm = quotient(t, p.by_tiles_n);
+    const int n = (t - tm * p.tiles_n) * TNF + wn * 32 * JN + fc * 8;
+    const long long r0 = (long long)tm * TM + wm * 32 * IM + trow;
+    const int left = n < p.N ? (int)min(p.rows - r0, (long long)TM) : 0;  // tokens from r0 on
+    TokenWalk<uint64_t> out_at, ahead;
+    out_at.start(p.om, r0);
+    out_at.off += feat_bytes<uint64_t>(p.om, n < p.N ? n : 0);
+    ahead = out_at;
+    const char* const aux = reinterpret_cast<const char*>(p.aux);
     u32x4 saved[2][32 / RPI];
     auto fetch = [&](int i, u32x4 (&to)[32 / RPI]) __attribute__((always_inline)) {
 #pragma unroll
       for (int q = 0; q < 32 / RPI; ++q) {
-        const bool there = r0 + i * 32 + RPI * q < p.rows && n < p.N;  // what is not there is not used either
-        to[q] = *reinterpret_cast<const u32x4*>(p.aux + (there ? ahead.part(p.om) + fo : 0));
-        ahead.advance(p.om, RPI);
+        to[q] = *reinterpret_cast<const u32x4*>(aux + (i * 32 + RPI * q < left ? ahead.off : 0));  // what is not there is not used either
+        ahead.advance(RPI);
       }
     };
     if (READS) fetch(0, saved[0]);
@@ -321,25 +381,32 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_nt_ke
         piece[q] = *reinterpret_cast<const u32x4*>(block + (trow + RPI * q) * SH::OUT_PITCH + fc * 16);
 #pragma unroll
       for (int q = 0; q < 32 / RPI; ++q) {
-        if (r0 + i * 32 + RPI * q < p.rows && n < p.N) {
-          const long long at = rwk.part(p.om) + fo;
+        if (i * 32 + RPI * q < left) {
           u32x4 y = piece[q];
           if (READS) {
             if (p.epi == EPI_DGELU) y = map8(y, saved[i & 1][q], [](float g, float h) { return g * dgelu_f(h); });
             else y = map8(y, saved[i & 1][q], [](float a, float b) { return a + b; });
           } else if (p.epi == EPI_GELU) {
-            *reinterpret_cast<u32x4*>(p.aux + at) = map8(y, y, [](float h, float) { return gelu_f(h); });
+            *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(p.aux) + out_at.off) = map8(y, y, [](float h, float) { return gelu_f(h); });
           }
-          *reinterpret_cast<u32x4*>(p.out + at) = y;
+          *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(p.out) + out_at.off) = y;
         }
-        rwk.advance(p.om, RPI);
+        out_at.advance(RPI);
       }
     }
   };
 
   const bool tail = p.K % BK != 0;
+  // the next stage of the stream, over the end of a tile too
+  auto advance = [&]() {
+    if (++ld_ks < nk) return true;
+    if (ld_tile + 1 == my_tiles) return false;
+    enter_tile();
+    return true;
+  };
   enter_tile();
   issue(0);
+  bool more = true;
   int buf = 0;
   for (int ti = 0; ti < my_tiles; ++ti) {
     for (int ks = 0; ks < nk; ++ks) {
@@ -348,12 +415,11 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_nt_ke
       if (ks == 0 && tid < TNF) lds_bias[(ti & 1) * TNF + tid] = jg::bf16_to_f32(bias_next);
       __syncthreads();  // stage ks is in LDS, and every wavefront is done with the other buffer
       if (ks == 0) init_acc(ti & 1);
-      if (++ld_ks < nk) issue(buf ^ 1);
-      else if (ld_tile + 1 < my_tiles) {
-        enter_tile();
-        issue(buf ^ 1);
+      if (more && (more = advance())) {
+        if (SPREAD) enter_stage();
+        else issue(buf ^ 1);
       }
-      compute(buf);
+      compute(buf, SPREAD && more ? buf ^ 1 : -1);
       buf ^= 1;
     }
     __syncthreads();  // the other wavefronts are done with the stage the results pass through
@@ -366,6 +432,7 @@ template <int IM, int JN, int WM, int WN>
 int launch_nt(NtParams& p, hipStream_t s, const char* who) {
   typedef NtShape<IM, JN, WM, WN> SH;
   p.tiles_n = jg::cdiv(p.N, SH::TNF);
+  p.by_tiles_n = div_by(p.tiles_n);
   const long long tiles = (long long)jg::cdiv(p.rows, SH::TM) * p.tiles_n;
   JG_REQUIRE(tiles < (1ll << 30), "%s: too many tiles", who);
   p.tiles = (int)tiles;
@@ -392,6 +459,7 @@ struct TnParams {
   long long rows;
   int N, C;
   int tiles_c, tiles;  // column tiles, all tiles; a workgroup is split * tiles + tile_n * tiles_c + tile_c
+  Div by_tiles_c, by_tiles;
   int stages_per_split;
 };
 
@@ -399,38 +467,13 @@ struct TnParams {
 template <int IM, int JN, int WM, int WN>
 struct TnShape {
   static constexpr int T = 32 * IM * WM;
-  static_assert(T == 32 * JN * WN && IM == WN, "square tile; block i of the bias gradient goes to wavefront column i");
+  static_assert(T == 32 * JN * WN && IM <= WN, "square tile; block i of the bias gradient goes to wavefront column i");
   static constexpr int WAVES = WM * WN, THREADS = 64 * WAVES;
   static constexpr int ROWB = 2 * T;                  // bytes of a token's row in LDS
   static constexpr int OP = BR * ROWB, STAGE = 2 * OP, LDS = 2 * STAGE;
   static constexpr int CPR = T / 8, RPI = 64 / CPR;   // 16-byte chunks per row, rows per transfer
   static constexpr int DMA = OP / 1024 / WAVES;       // transfers of a wavefront per operand and stage
   static constexpr int JROWS = WAVES * RPI;           // rows between a wavefront's transfers
-};
-
-// Tokens r, r + step, ... of an operand as byte offsets; heads: (b * H * S + s) * D, row-major: r * ld.
-// OFF: uint32_t, or uint64_t where an operand has 2^32 bytes or more.
-template <typename OFF>
-struct TokenWalk {
-  OFF off;         // bytes
-  int s, S;        // position in the batch entry and its length
-  OFF row, jump;   // bytes between tokens of an entry; extra bytes from the end of an entry to the next one
-  __device__ __forceinline__ void start(const Map& m, long long r) {
-    row = (OFF)(m.heads ? m.D : m.ld) * 2u;
-    S = m.heads ? m.S : 0x7fffffff;
-    jump = m.heads ? (OFF)(m.H - 1) * (OFF)m.S * row : 0u;
-    const long long b = m.heads ? r / m.S : 0;
-    s = m.heads ? (int)(r - b * S) : 0;
-    off = (OFF)(row_part(m, r) * 2);
-  }
-  __device__ __forceinline__ void advance(int by) {
-    s += by;
-    off += (OFF)by * row;
-    while (s >= S) {  // at most once where an entry is longer than the step
-      s -= S;
-      off += jump;
-    }
-  }
 };
 
 // Weight gradient. The tiles of g and x (64 tokens x T features) lie in LDS as they lie in memory, a token per row,
@@ -440,6 +483,11 @@ struct TokenWalk {
 // instruction transposes: with its reduction 72 us for 32768 tokens, 1536 x 512 (101 us with both and a round more), 1132 us for
 // 8192 x 8192 x 8192 (1294). A batch entry may be of any length: the octet-wise staging took multiples of 8 tokens
 // only and left the rest to the FMA kernel (5 x 590 tokens, 896 features, qkv and output projection: 2247 -> 250 us). The bias gradient is one more matrix instruction with ones, in the first column of tiles.
+// Around the stages: the tokens of a stage that lie a row apart share their offsets' products (walked token by token they were 0.3 of
+// 0.75 us a stage), the partials leave by pointers that walk the rows (by index 2.6 us, 0.9 now), and tn_plan sets how many there are.
+// us before -> now with the reduction: 924 tokens, 768 x 768 21.2 -> 13.6, 2560, 640 x 160 14.4 -> 10.9, 2680, 2688 x 896 37.7 -> 28.9, 32768,
+// 512 x 512 42.4 -> 32.7, 65536, 512 x 128 26.3 -> 25.2. (A ring of four stages changed nothing, transfers between the matrix instructions, as in
+// proj_nt_kernel, cost 5 % where the operands stream from memory.)
 // OFF as in TokenWalk: 64-bit offsets from 2^32 bytes an operand on, at the same rate (2048 x 512 over 2^20 tokens 2.44 ms,
 // 2040 x 512 with 32-bit ones 2.48; the FMA kernel, which the larger one would else fall to, 238 ms).
 template <int IM, int JN, int WM, int WN, typename OFF>
@@ -459,8 +507,8 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
     const int per_xcd = gridDim.x / 8;
     if (id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
   }
-  const int split = id / p.tiles, tile = id - split * p.tiles;
-  const int tile_c = tile % p.tiles_c, tile_n = tile / p.tiles_c;
+  const int split = quotient(id, p.by_tiles), tile = id - split * p.tiles;
+  const int tile_n = quotient(tile, p.by_tiles_c), tile_c = tile - tile_n * p.tiles_c;
   const int n0 = tile_n * T, c0 = tile_c * T;
   const long long r_first = (long long)split * p.stages_per_split * BR;
   long long r_last = r_first + (long long)p.stages_per_split * BR;
@@ -471,36 +519,41 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
   const int my_row = wave * SH::RPI + lane / SH::CPR;
   const int chunk = (lane % SH::CPR) ^ ((my_row & 3) << 2);  // JROWS is a multiple of 4: the same for every j
   // a chunk past the last feature repeats the last one and is dropped
-  const OFF gf = (OFF)(feat_part(p.gm, min(n0 + chunk * 8, p.N - 8)) * 2);
-  const OFF xf = (OFF)(feat_part(p.xm, min(c0 + chunk * 8, p.C - 8)) * 2);
-  TokenWalk<OFF> gw, xw;
-  gw.start(p.gm, min(r_first + my_row, p.rows - 1));
-  xw.start(p.xm, min(r_first + my_row, p.rows - 1));
+  const OFF gf = feat_bytes<OFF>(p.gm, min(n0 + chunk * 8, p.N - 8));
+  const OFF xf = feat_bytes<OFF>(p.xm, min(c0 + chunk * 8, p.C - 8));
+  const OFF g_row = (OFF)(p.gm.heads ? p.gm.D : p.gm.ld) * 2u, x_row = (OFF)(p.xm.heads ? p.xm.D : p.xm.ld) * 2u;
+  const OFF g_lane = (OFF)my_row * g_row + gf, x_lane = (OFF)my_row * x_row + xf;
+  // S = 0: the tokens of an operand lie a row apart throughout
+  const int S = p.gm.heads ? p.gm.S : p.xm.heads ? p.xm.S : 0;
+  const Div by_S = p.gm.heads ? p.gm.by_S : p.xm.by_S;
   const uint32_t lds_g = jg::lds_address(smem) + wave_u * 1024;
+  auto entry_of = [&](long long r) { return sizeof(OFF) == 4 ? (long long)quotient((uint32_t)r, by_S) : r / S; };  // batch entry of a token
+  auto row_at = [&](const Map& m, long long b, long long r) {  // first element of token r, which is of batch entry b
+    return m.heads ? (b * m.H * m.S + (r - b * m.S)) * m.D : r * m.ld;
+  };
   auto issue = [&](int st, int buf) {
-    const long long left = p.rows - (r_first + (long long)st * BR);
+    const long long first = r_first + (long long)st * BR, left = p.rows - first;
     const uint32_t dst = lds_g + buf * SH::STAGE;
-    if (left >= BR) {  // wave-uniform
-      TokenWalk<OFF> a = gw, b = xw;
+    const long long b = S == 0 ? 0 : entry_of(first);
+    if (left >= BR && (S == 0 || first - b * S + BR <= S)) {  // wave-uniform: the tokens of the stage lie a row apart
+      OFF g_at = g_lane + (OFF)(row_at(p.gm, b, first) * 2), x_at = x_lane + (OFF)(row_at(p.xm, b, first) * 2);
 #pragma unroll
       for (int j = 0; j < SH::DMA; ++j) {
-        jg::to_lds_1k(p.g, a.off + gf, dst + j * SH::WAVES * 1024);
-        jg::to_lds_1k(p.x, b.off + xf, dst + SH::OP + j * SH::WAVES * 1024);
-        a.advance(SH::JROWS);
-        b.advance(SH::JROWS);
+        jg::to_lds_1k(p.g, g_at, dst + j * SH::WAVES * 1024);
+        jg::to_lds_1k(p.x, x_at, dst + SH::OP + j * SH::WAVES * 1024);
+        g_at += SH::JROWS * g_row;
+        x_at += SH::JROWS * x_row;
       }
-      gw = a;
-      xw = b;
-    } else {  // the stage the tokens end in: a row past the end repeats the last token and is cleared below
+    } else {  // a batch entry ends in the stage, or the tokens do: a row past the end repeats the last token and is cleared below
 #pragma unroll
       for (int j = 0; j < SH::DMA; ++j) {
-        const long long r = min(r_first + (long long)st * BR + j * SH::JROWS + my_row, p.rows - 1);
-        jg::to_lds_1k(p.g, (OFF)(row_part(p.gm, r) * 2) + gf, dst + j * SH::WAVES * 1024);
-        jg::to_lds_1k(p.x, (OFF)(row_part(p.xm, r) * 2) + xf, dst + SH::OP + j * SH::WAVES * 1024);
+        const long long r = min(first + j * SH::JROWS + my_row, p.rows - 1), e = S == 0 ? 0 : entry_of(r);
+        jg::to_lds_1k(p.g, (OFF)(row_at(p.gm, e, r) * 2) + gf, dst + j * SH::WAVES * 1024);
+        jg::to_lds_1k(p.x, (OFF)(row_at(p.xm, e, r) * 2) + xf, dst + SH::OP + j * SH::WAVES * 1024);
       }
     }
   };
-  static_assert(SH::DMA * SH::JROWS == BR, "the walkers stand at the next stage after their transfers");
+  static_assert(SH::DMA * SH::JROWS == BR, "whole stages");
   auto clear_tail = [&](int st, int buf) {
     const long long left = p.rows - (r_first + (long long)st * BR);
     if (left >= BR) return;
@@ -525,7 +578,7 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
   for (int i = 0; i < IM; ++i) g_off[i] = frag_off(wn * IM + i);
 #pragma unroll
   for (int j = 0; j < JN; ++j) x_off[j] = SH::OP + frag_off(wc * JN + j);
-  const int b_off = frag_off(wn * IM + wc);  // the block whose bias gradient this wavefront sums
+  const int b_off = frag_off(wn * IM + min(wc, IM - 1));  // the block whose bias gradient this wavefront sums
   auto tr_frag = [&](const unsigned char* at) {
     typedef short i16x4 __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) i16x4* tr_ptr;
@@ -545,9 +598,10 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
 #pragma unroll
   for (int e = 0; e < 8; ++e) ones[e] = (__bf16)1.0f;
 
+  constexpr int AHEAD = IM * JN <= 4 ? 2 : 1;  // steps of 16 tokens between a fragment's request and its use
   auto compute = [&](int buf, auto with_bias) {
     const unsigned char* st = smem + buf * SH::STAGE;
-    bf16x8 fr[2][IM + JN + 1];
+    bf16x8 fr[AHEAD + 1][IM + JN + 1];
     auto fetch = [&](int kk, bf16x8 (&f)[IM + JN + 1]) {
       const unsigned char* at = st + kk * 16 * ROWB;
 #pragma unroll
@@ -556,17 +610,19 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
       for (int t = 0; t < JN; ++t) f[IM + t] = tr_frag(at + x_off[t]);
       if (with_bias) f[IM + JN] = tr_frag(at + b_off);
     };
-    fetch(0, fr[0]);
+#pragma unroll
+    for (int kk = 0; kk < AHEAD; ++kk) fetch(kk, fr[kk]);
 #pragma unroll
     for (int kk = 0; kk < BR / 16; ++kk) {
-      if (kk + 1 < BR / 16) fetch(kk + 1, fr[(kk + 1) & 1]);
+      if (kk + AHEAD < BR / 16) fetch(kk + AHEAD, fr[(kk + AHEAD) % (AHEAD + 1)]);
+      const bf16x8(&f)[IM + JN + 1] = fr[kk % (AHEAD + 1)];
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < IM; ++i)
 #pragma unroll
         for (int j = 0; j < JN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[kk & 1][i], fr[kk & 1][IM + j], acc[i][j], 0, 0, 0);
-      if (with_bias) acc_b = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[kk & 1][IM + JN], ones, acc_b, 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[i], f[IM + j], acc[i][j], 0, 0, 0);
+      if (with_bias) acc_b = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[IM + JN], ones, acc_b, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -586,21 +642,29 @@ __global__ __launch_bounds__(64 * WM * WN, IM * JN >= 8 ? 1 : 2) void proj_tn_ke
   else run(std::false_type{});
 
   // register e of block (i, j): row n0 + (wn*IM + i)*32 + 8*(e/4) + 4*kg + e%4, column c0 + (wc*JN + j)*32 + ln
-  float* part = p.part + (size_t)split * p.N * p.C;
+  {
+    const int n_first = n0 + wn * IM * 32 + kg * 4, c_first = c0 + wc * JN * 32 + ln;
+    const int rows_left = p.N - n_first, cols_left = p.C - c_first;
+    auto store = [&](auto whole) __attribute__((always_inline)) {
+      float* at = p.part + (size_t)split * p.N * p.C + (size_t)n_first * p.C + c_first;
 #pragma unroll
-  for (int i = 0; i < IM; ++i)
+      for (int i = 0; i < IM; ++i)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int n = n0 + (wn * IM + i) * 32 + (e >> 2) * 8 + kg * 4 + (e & 3);
-      if (n < p.N) {
+        for (int e4 = 0; e4 < 4; ++e4) {
 #pragma unroll
-        for (int j = 0; j < JN; ++j) {
-          const int cidx = c0 + (wc * JN + j) * 32 + ln;
-          if (cidx < p.C) part[(size_t)n * p.C + cidx] = acc[i][j][e];
+          for (int e = 0; e < 4; ++e) {
+#pragma unroll
+            for (int j = 0; j < JN; ++j)
+              if (whole || (i * 32 + e4 * 8 + e < rows_left && j * 32 < cols_left)) at[j * 32] = acc[i][j][e4 * 4 + e];
+            at += p.C;
+          }
+          at += 4 * (size_t)p.C;
         }
-      }
-    }
-  if (want_bias && ln == 0) {  // every column of acc_b holds the same sums
+    };
+    if (n0 + T <= p.N && c0 + T <= p.C) store(std::true_type{});  // uniform over the workgroup
+    else store(std::false_type{});
+  }
+  if (want_bias && wc < IM && ln == 0) {  // every column of acc_b holds the same sums
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int n = n0 + (wn * IM + wc) * 32 + (e >> 2) * 8 + kg * 4 + (e & 3);
@@ -822,6 +886,7 @@ int make_map(Map* m, int heads, long long features, long long rows, int B, int H
   m->heads = heads ? 1 : 0;
   m->ld = features;
   m->B = B; m->H = H; m->S = S; m->D = D;
+  m->by_S = div_by(S); m->by_D = div_by(D); m->by_H = div_by(H);
   if (!heads) return JG_OK;
   JG_REQUIRE(B > 0 && H > 0 && S > 0 && D > 0, "%s: %s: heads layout needs positive B, H, S, D", who, what);
   JG_REQUIRE((long long)B * S == rows, "%s: %s: B * S = %lld does not match %lld tokens", who, what,
@@ -837,48 +902,51 @@ bool map_vec_ok(const Map& m, long long features) {
   if (features % 8 != 0) return false;
   return m.heads ? (m.D % 8 == 0) : (m.ld % 8 == 0);
 }
-// Tile edge of the weight-gradient kernel: 256 (half the operand traffic per MFMA, one workgroup
-// per compute unit) when such tiles and their splits still fill most of the chip, else 128. A split (a range of
-// tokens) is worth its partial tile from about 8 stages on.
-constexpr int TN_MOST_SPLITS = 64;
 long long tn_stages(long long rows) { return (rows + BR - 1) / BR; }
-int tn_tile(long long rows, int n, int c) {
-  if (n < 256 || c < 256) return 128;
-  const long long tiles = (long long)jg::cdiv(n, 256) * jg::cdiv(c, 256);
-  const long long most = tn_stages(rows) / 8;
-  return tiles * (most < 1 ? 1 : most < TN_MOST_SPLITS ? most : TN_MOST_SPLITS) >= jg::cu_count() * 3 / 4 ? 256 : 128;
-}
-// Token ranges the contraction is cut into so that the tiles fill the chip.
-int tn_splits(long long rows, int n, int c) {
-  const int t = tn_tile(rows, n, c);
-  const long long tiles = (long long)jg::cdiv(n, t) * jg::cdiv(c, t), stages = tn_stages(rows), cus = jg::cu_count();
-  if (t == 256) {
-    // One workgroup fits a compute unit, so a few more than these (256) cost a second round: 12 tiles in 22 splits
-    // (1536 x 512 over 32768 tokens) took 88 us, in 21 splits 72. The number of splits with the least of: rounds of
-    // workgroups times the stages of a split (1.7 us each, 5 us around them), and the partials, written and read back at about
-    // 6 TB/s. 3072 x 1024 over 8192 tokens 102 -> 74 us (6 -> 5 splits), 2112 x 704 over 20000 125 -> 91 us (10 -> 9),
-    // 512 x 512 over 32768 44 -> 41 us (64 -> 47).
-    int best = 1;
-    double least = 0.0;
-    for (int k = 1; k <= TN_MOST_SPLITS && (k == 1 || k <= stages / 8); ++k) {
-      const double rounds = (double)((tiles * k + cus - 1) / cus), walk = (double)((stages + k - 1) / k);
-      const double us = rounds * (walk * 1.7 + 5.0) + k * (double)n * c * 8.0 / 6.0e6;
-      if (k == 1 || us < least) {
-        least = us;
-        best = k;
+
+// Tile edge of the weight-gradient kernel and the ranges of tokens (splits) the contraction is cut into: the pair with the least of
+// what the figures of both say, us on 256 compute units (measured, the reduction included, and what the rule expects):
+//   128   a stage takes 0.7 where a compute unit has one workgroup, 1 where some have two, and all of them together no less than
+//         14.6 TB/s out of the caches allow; 5.4 around them. 32768 tokens, 512 x 512, 16 splits 32.3 (33.4), 32 33.7 (35.0), 1536 x 512, 8 splits
+//         75.9 (77.8), 10 70.7 (71.0); 5000, 1024 x 1024, 4 splits 24.8 (25.0), 8 28.5 (27.9); 924, 768 x 768, 1 split 17.2 (16.9), 3 12.9 (11.3).
+//   256   half the operand traffic per matrix instruction and one workgroup a compute unit: 1.7 a stage and 5 a round of workgroups.
+//         8192 tokens, 3072 x 1024, 5 splits 70.7 (70.2; at 128 76.4), 32768 219 (201; at 128 238), 512 x 512, 48 splits 38.5 (40.5).
+// and the partials written and read back at 6 TB/s. More splits only where they win a twentieth with the partials counted half as
+// much again: a Swin block holds those of all its weights until the end of its backward. With at least eight stages a split, and 256 wherever
+// its tiles filled most of the chip, 924 tokens, 768 x 768 took 17.1, 5000, 1024 x 1024 32.2, 32768, 512 x 512 39.7.
+constexpr int TN_MOST_SPLITS = 64;
+struct TnPlan {
+  int tile, splits;
+};
+TnPlan tn_plan(long long rows, int n, int c) {
+  const long long stages = tn_stages(rows), cus = jg::cu_count();
+  const double partial = (double)n * c * 8.0 / 6.0e6;
+  TnPlan best{128, 1};
+  double best_us = 0.0;
+  for (const int t : {128, 256}) {
+    if (t == 256 && (n < 256 || c < 256)) break;
+    const long long tiles = (long long)jg::cdiv(n, t) * jg::cdiv(c, t);
+    // (with one to three tiles as many as put a workgroup on every compute unit)
+    const long long most = std::min<long long>(stages, std::max<long long>(TN_MOST_SPLITS, cus / tiles));
+    double least = 0.0, us = 0.0;
+    int splits = 1;
+    for (long long k = 1; k <= most; k += 1 + k / 8) {
+      const long long walk = (stages + k - 1) / k, workgroups = tiles * k;
+      double sums;
+      if (t == 256) sums = (double)((workgroups + cus - 1) / cus) * (walk * 1.7 + 5.0);
+      else sums = std::max(walk * (workgroups <= cus ? 0.7 : (double)((workgroups + 2 * cus - 1) / (2 * cus))), (double)tiles * stages * 32768.0 / 14.6e6) + 5.4;
+      if (least == 0.0 || sums + 1.5 * k * partial < 0.95 * least) {
+        least = sums + 1.5 * k * partial;
+        us = sums + k * partial;
+        splits = (int)((stages + walk - 1) / walk);  // (no empty ones)
       }
     }
-    return best;
+    if (t == 128 || us < best_us) {
+      best = TnPlan{t, splits};
+      best_us = us;
+    }
   }
-  // 128: two workgroups a compute unit, two rounds of them; at most 64 splits, but with one to three tiles as many
-  // as put a workgroup on every compute unit: a compute unit streams its operands at some 20 GB/s, so 64 workgroups
-  // leave three quarters of the memory system idle (128 x 128 over 65536 tokens: 23 -> 13 us, the reduction 5 -> 6 us)
-  const long long cap = tiles * TN_MOST_SPLITS >= cus ? TN_MOST_SPLITS : cus / tiles;
-  long long want = (4 * cus + tiles - 1) / tiles;
-  if (want > stages / (cap > TN_MOST_SPLITS ? 4 : 8)) want = stages / (cap > TN_MOST_SPLITS ? 4 : 8);
-  if (want < 1) want = 1;
-  if (want > cap) want = cap;
-  return (int)want;
+  return best;
 }
 
 template <int IM, int JN, int WM, int WN, typename OFF>
@@ -886,6 +954,8 @@ int launch_tn(TnParams& p, int splits, hipStream_t s, const char* who) {
   typedef TnShape<IM, JN, WM, WN> SH;
   p.tiles_c = jg::cdiv(p.C, SH::T);
   p.tiles = jg::cdiv(p.N, SH::T) * p.tiles_c;
+  p.by_tiles_c = div_by(p.tiles_c);
+  p.by_tiles = div_by(p.tiles);
   void (*kern)(TnParams) = &proj_tn_kernel<IM, JN, WM, WN, OFF>;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS) != hipSuccess)
     JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, SH::LDS);
@@ -948,14 +1018,21 @@ static int proj_nt_common(const char* who, void* out, void* aux, int epi, const 
   p.out = static_cast<uint16_t*>(out);
   p.am = am; p.om = om;
   p.rows = rows; p.N = n_out; p.K = k_in;
-  // 256 x 256 tiles (half the operand traffic per MFMA) once they fill the chip, else 128 x 128
-  const long long big_tiles = (long long)jg::cdiv(rows, 256) * jg::cdiv(n_out, 256);
-  // the 256-wide tile only where its last column of tiles is more than half full
+  // Tiles of 256 x 256 (half the operand traffic per MFMA), one workgroup a compute unit, where their rounds leave no more than two fifths of
+  // the chip idle and the last column of tiles is more than half full; below a round only contractions of 1024 and more gain (us, 256 : 128:
+  // 16000 tokens, 1024 -> 1024 34.6 : 39.8, 5000, 1024 -> 2048 30.3 : 33.8, 8000, 384 -> 768 14.9 : 10.8; 282 tiles, 12000, 512 -> 1536
+  // 33.4 : 28.3; 512, 32768, 256 -> 1024 26.8 : 28.1). What is read on the way out and short contractions, which are little but their
+  // epilogue, are better off with two workgroups a compute unit (y gelu'(aux), 65536, 128 -> 512 42.3 : 38.7, 55680, 256 -> 1024 91.2 : 86.8;
+  // plain, 65536, 128 -> 512 21.5 : 19.6; with GELU, whose arithmetic bounds it, 250000, 128 -> 512 150 : 183).
+  const long long cus = jg::cu_count(), tiles_256 = (long long)jg::cdiv(rows, 256) * jg::cdiv(n_out, 256);
   const int waste = jg::cdiv(n_out, 256) * 256 - n_out;
-  if (big_tiles >= jg::cu_count() && waste < 128) return launch_nt<4, 2, 2, 4>(p, s, who);
-  // 64 x 64 where 128 x 128 tiles would leave most of the chip idle (468 tokens, 704 -> 2112: 7.9 us, 13.1 before)
-  if ((long long)jg::cdiv(rows, 128) * jg::cdiv(n_out, 128) < jg::cu_count() / 2) return launch_nt<1, 1, 2, 2>(p, s, who);
-  return launch_nt<2, 2, 2, 2>(p, s, who);
+  const bool fills = tiles_256 * 5 >= (tiles_256 + cus - 1) / cus * cus * 3 && (tiles_256 >= cus || k_in >= 1024);
+  const bool epilogue_only = epi == EPI_DGELU ? k_in <= 256 : epi != EPI_GELU && k_in <= 128;
+  if (fills && waste < 128 && !epilogue_only) return launch_nt<4, 2, 2, 4>(p, s, who);
+  // 64 x 64 where 128 x 128 tiles would leave a quarter of the chip idle (us, 64 : 128: 468 tokens, 704 -> 2112 7.2 : 9.7, 924, 768 -> 2304
+  // 9.6 : 12.2, 4000, 640 -> 640 8.9 : 9.7; 224 tiles of 128, 3520, 256 -> 1024 7.5 : 6.9)
+  if ((long long)jg::cdiv(rows, 128) * jg::cdiv(n_out, 128) < cus * 3 / 4) return launch_nt<1, 1, 2, 2>(p, s, who);
+  return launch_nt<2, 1, 2, 4>(p, s, who);
 }
 
 int jg_proj_nt(void* out, const void* a, const void* w, const void* bias, int dtype, int64_t rows, int n_out,
@@ -1019,7 +1096,7 @@ int jg_transpose16(void* dst, const void* src, int64_t rows, int64_t cols, void*
 
 size_t jg_proj_tn_workspace(int64_t rows, int n, int c) {
   if (rows <= 0 || n <= 0 || c <= 0) return 0;
-  const size_t splits = (size_t)tn_splits(rows, n, c);
+  const size_t splits = (size_t)tn_plan(rows, n, c).splits;
   return splits * ((size_t)n * c + n) * sizeof(float);
 }
 
@@ -1067,16 +1144,17 @@ static int proj_tn_common(const char* who, jg_reductions* later, void* gw, void*
   p.x = static_cast<const uint16_t*>(x);
   p.gm = gm; p.xm = xm;
   p.rows = rows; p.N = n; p.C = c;
-  const int splits = tn_splits(rows, n, c);
+  const TnPlan plan = tn_plan(rows, n, c);
+  const int splits = plan.splits;
   const long long stages = (rows + BR - 1) / BR;
   p.stages_per_split = (int)((stages + splits - 1) / splits);
   p.part = static_cast<float*>(workspace);
   p.bias_part = gb != nullptr ? p.part + (size_t)splits * n * c : nullptr;
   const bool far = (unsigned long long)rows * (n > c ? n : c) >= (1ull << 31);
-  if (tn_tile(rows, n, c) == 256)
+  if (plan.tile == 256)
     rc = far ? launch_tn<4, 2, 2, 4, uint64_t>(p, splits, s, who) : launch_tn<4, 2, 2, 4, uint32_t>(p, splits, s, who);
   else
-    rc = far ? launch_tn<2, 2, 2, 2, uint64_t>(p, splits, s, who) : launch_tn<2, 2, 2, 2, uint32_t>(p, splits, s, who);
+    rc = far ? launch_tn<1, 2, 4, 2, uint64_t>(p, splits, s, who) : launch_tn<1, 2, 4, 2, uint32_t>(p, splits, s, who);
   if (rc) return rc;
   if (later != nullptr && out32) {
     rc = jg::add_reduction(later, jg::RED_SLICES, splits, (int64_t)n * c, p.part, static_cast<float*>(gw), nullptr);

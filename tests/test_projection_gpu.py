@@ -304,6 +304,7 @@ def test_transpose_is_exact(n, k, dtype, dev):
 @pytest.mark.parametrize("b,s,c,n_out,heads", [
     (1, 1, 8, 24, 1), (3, 5, 64, 192, 2), (2, 63, 72, 200, 1), (5, 117, 136, 264, 3), (1, 65, 64, 64, 2), (7, 129, 256, 512, 4),
     (2, 4100, 512, 1536, 8), (9, 1001, 264, 768, 4),
+    (5, 3201, 1272, 1240, 2), (5335, 3, 1272, 1240, 2),  # tiles of 256 x 256 each way, entries that end inside one and far shorter ones
 ], ids=str)
 def test_gemm_tiles_with_remainders(b, s, c, n_out, heads, dev):
     """Token counts beside the 64-token stages, batch entries that end inside a stage (and are shorter than one),
