@@ -85,6 +85,16 @@ static_assert(2 * IN_ROWS <= WAVES * (LANES_ODD / OCTS), "every row of tasks has
 
 __device__ __forceinline__ int in_slot(int col) { return (col & 7) * OCTS + (col >> 3); }
 
+// A tile's place from its number: three to five divisions, twice a tile and all of it in front of a workgroup's first load. The compiler's
+// own (and one more, and a remainder of ragged channels by two of them in every stage) were 1.5 to 2 us of a workgroup with a tile or two.
+// Read from the kernel-argument segment where it is wanted (walk_of): held from the kernel's start on, it pushes the stage loop's
+// scalar registers out. Forward / gradient with the fold: 2 x 40 -> 72 of 217 x 301 31.4 -> 29.6 us / the same, 4 x 7 -> 91 of 163 x 957
+// 67.6 -> 62.7 / 64.4 -> 60.5, 1 x 17 -> 24 of 50 x 76 x 26 23.2 -> 21.7 / 41.8 -> 39.6, 2 x 32 -> 32 of 128^3 280 -> 277 / 378 -> 367.
+struct TileWalk {
+  jg::Div by_plane, by_tw, by_od, by_wgs;  // tiles of a plane, tile columns, produced planes, workgroups of an XCD
+  int per_plane, tiles_w, Dout;
+};
+
 struct FwdParams {
   const uint16_t* x;    // (N, C, Din, Hin, Win) bf16: the tensor that is convolved
   const char* x_end;    // one past the last byte of x
@@ -114,7 +124,7 @@ struct FwdParams {
   // The first extra_h produced rows and extra_w columns (0, or pad_h / pad_w; org_w is then the same) lie above and left of the
   // tile grid: the workgroups at tile row / column 0 make them beside their tile, see compute_left and compute_top.
   int extra_h, extra_w;
-  int sw;               // tile order inside a plane: row-major inside bands of sw tile columns, band after band
+  TileWalk walk;
   int total_tiles;      // N * Dout * tiles_h * tiles_w
   int nc16;             // KD * Cp / 16
   int wc16;             // 16-channel steps whose weights sit in LDS at a time (a group)
@@ -147,6 +157,16 @@ __device__ __forceinline__ void* strip_entry(int idx) {
   (void)idx;
   return nullptr;
 #endif
+}
+
+__device__ __forceinline__ TileWalk walk_of() {
+  typedef const __attribute__((address_space(4))) TileWalk* Arg;
+  Arg arg = nullptr;
+#if defined(__HIP_DEVICE_COMPILE__)
+  arg = reinterpret_cast<Arg>(reinterpret_cast<uintptr_t>((void*)__builtin_amdgcn_kernarg_segment_ptr()) + sizeof(StripTable) + offsetof(FwdParams, walk));
+  asm volatile("" : "+s"(arg));
+#endif
+  return {{arg->by_plane.m, arg->by_plane.s}, {arg->by_tw.m, arg->by_tw.s}, {arg->by_od.m, arg->by_od.s}, {arg->by_wgs.m, arg->by_wgs.s}, arg->per_plane, arg->tiles_w, arg->Dout};
 }
 
 // ---------------------------------------------------------------- weight prep
@@ -400,7 +420,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   const int t_len = t_end - t_begin;
   if (slot_in_xcd >= t_len) return;
   const int t_rot = (int)(((long long)xcd * t_len) >> 3);
-  const int my_tiles = (t_len - slot_in_xcd + wg_per_xcd - 1) / wg_per_xcd;
+  const int my_tiles = jg::quotient(t_len - slot_in_xcd + wg_per_xcd - 1, p.walk.by_wgs);
   auto tile_of = [&](int ti) {  // ti-th tile of this workgroup
     int i = slot_in_xcd + ti * wg_per_xcd + t_rot;
     if (i >= t_len) i -= t_len;
@@ -509,32 +529,30 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   const char* stg_origin = nullptr;  // its origin (wave-uniform)
   uint32_t stg_mask = 0xffu;  // this task's pixels inside the tensor (one bit each), where stg_masked; bit 8: not loaded yet
   uint32_t stg_odd = 0;       // not EVEN: one bit per channel, the task starts on the upper half of a dword
+  int stg_left = 0;           // channels from the staged step's first one to the end (wave-uniform)
 
   struct TileCoord {
     int n, od, th, tw;
   };
   auto coord = [&](int tile) {
     TileCoord c;
-    const int per_plane = p.tiles_h * p.tiles_w;
-    int tq = tile / per_plane;
-    int j = tile - tq * per_plane;
+    const TileWalk w = walk_of();
+    const int tq = jg::quotient(tile, w.by_plane);
+    int j = tile - tq * w.per_plane;
     // With columns or rows beside the grid the tiles at its edge have more to do. The tiles of a plane are turned by one from plane to
     // plane and its columns from row to row: a workgroup, whose steps are whole rows or whole planes, would else stay at one
     // place of every plane for its life (2 x 32 -> 32 of 128^3 384 -> 339 us), and in one column, where the rows of a power of two
     // alias in L2 (8 x 64 -> 64 of 1024 x 1024 931 -> 829 us).
-    if (RIM) j = (j + tq) % per_plane;
-    const int band = p.tiles_h * p.sw;          // tiles in a full band
-    const int b = j / band;                     // band number; the last one may be narrower
-    j -= b * band;
-    const int width = min(p.sw, p.tiles_w - b * p.sw);
-    c.th = j / width;
-    c.tw = b * p.sw + (j - c.th * width);
+    if (RIM) j += tq - jg::quotient(tq, w.by_plane) * w.per_plane;
+    if (RIM && j >= w.per_plane) j -= w.per_plane;
+    c.th = jg::quotient(j, w.by_tw);
+    c.tw = j - c.th * w.tiles_w;
     if (RIM) {
-      c.tw += c.th % p.tiles_w;
-      if (c.tw >= p.tiles_w) c.tw -= p.tiles_w;
+      c.tw += c.th - jg::quotient(c.th, w.by_tw) * w.tiles_w;
+      if (c.tw >= w.tiles_w) c.tw -= w.tiles_w;
     }
-    c.od = tq % p.Dout;
-    c.n = tq / p.Dout;
+    c.n = jg::quotient(tq, w.by_od);
+    c.od = tq - c.n * w.Dout;
     return c;
   };
 
@@ -591,7 +609,8 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     // Channels of this task that exist (all 8 unless C is not a multiple of 16). The vector
     // path below reads the others anyway (they lie inside the tensor: the interior test covers
     // all 16 channel planes) and store_stage zeroes them; the guarded paths skip them.
-    const int cvalid = p.C - c0 - g8 * 8;
+    stg_left = p.C - c0;
+    const int cvalid = stg_left - g8 * 8;
     const int id = cur.od + kd - p.pad_d;
     const int ih0 = cur.ih0, iw0 = cur.iw0;
     const bool depth_ok = id >= 0 && id < p.Din;
@@ -699,13 +718,13 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     }
   };
 
-  auto store_stage = [&](int buf, int stage) {  // stage: counted over this workgroup's tiles
+  auto store_stage = [&](int buf) {
     if (!has_task) return;
     if (stg_masked && __builtin_amdgcn_ballot_w64((stg_mask & 0x100u) != 0) != 0) {
       // a task whose bytes reach over the tensor's ends (the first and last rows of the first and last channel):
       // dword by dword, those that hold a pixel of the tensor
       if ((stg_mask & 0x100u) != 0) {
-        const int cvalid = p.C - ((stage % p.nc16) * CK) % p.Cp - g8 * 8;
+        const int cvalid = stg_left - g8 * 8;
         const char* a = stg_origin + t_off;
         stg_odd = 0;
 #pragma unroll
@@ -720,7 +739,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
       }
     }
     if (p.Cp != p.C) {  // uniform: zero the channels of this step that do not exist
-      const int cvalid = p.C - ((stage % p.nc16) * CK) % p.Cp - g8 * 8;
+      const int cvalid = stg_left - g8 * 8;
 #pragma unroll
       for (int c = 0; c < 8; ++c)
         if (c >= cvalid) {
@@ -1539,7 +1558,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   } else if (p.ngroups == 1) {
     load_weights(0);
   }
-  store_stage(0, 0);
+  store_stage(0);
   transfers_landed();
   if (stages > 1) issue_stage();
   __syncthreads();
@@ -1573,7 +1592,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
       const bool after_epilogue = epilogue_uses_lds && c16 == 0 && ti > 0;
       const bool stage_now = stage_early && !after_epilogue;
       if (stage_now) {
-        if (q + 1 < stages) store_stage(buf ^ 1, q + 1);
+        if (q + 1 < stages) store_stage(buf ^ 1);
         if (q + 2 < stages) issue_stage();
       }
       if (live) {
@@ -1588,7 +1607,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
       // nothing to wait for, and the wavefronts that are through with their stores do not wait for the others here)
       if (after_epilogue) __syncthreads();
       if (!stage_now) {
-        if (q + 1 < stages) store_stage(buf ^ 1, q + 1);  // other buffer: no hazard with this stage's reads
+        if (q + 1 < stages) store_stage(buf ^ 1);  // other buffer: no hazard with this stage's reads
         if (q + 2 < stages) issue_stage();
       }
       if (live) {
@@ -1882,7 +1901,6 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
   p.lead = even ? (L.pad_w - p.org_w) & 1 : 0;
   p.tiles_h = (p.Hout - p.extra_h + TH - 1) / TH;
   p.tiles_w = (p.Wout - p.org_w + TW - 1) / TW;
-  p.sw = p.tiles_w;
   const long long tiles = (long long)L.N * L.Dout * p.tiles_h * p.tiles_w;
   JG_REQUIRE(tiles < (1ll << 30), "%s: too many tiles", who);
   p.total_tiles = (int)tiles;
@@ -1900,6 +1918,7 @@ int launch_conv(const Launch& L, void* ws, size_t ws_bytes, hipStream_t s, const
   if (tiles == 0) return JG_OK;
   const size_t lds = lay.lds_bytes;
   int wgs = workgroups_for(tiles, lay.mtiles);
+  p.walk = TileWalk{jg::div_by(p.tiles_h * p.tiles_w), jg::div_by(p.tiles_w), jg::div_by(p.Dout), jg::div_by((wgs + 7) / 8), p.tiles_h * p.tiles_w, p.tiles_w, p.Dout};
   dim3 grid((unsigned)wgs, (unsigned)lay.mtiles, 1);
   void (*kern)(StripTable, FwdParams) = nullptr;
   if (L.f16 && L.xt != nullptr)

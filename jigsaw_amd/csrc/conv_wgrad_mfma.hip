@@ -95,6 +95,8 @@ struct WgradParams {
   int pad_d, pad_h, pad_w;
   int row_pairs, col_tiles;
   long long total_stages;  // N * Dout * col_tiles * row_pairs
+  long long per;           // of them a workgroup takes
+  jg::Div by_rp, by_ct, by_od, by_pairs, by_ci;  // row_pairs, col_tiles, Dout, npairs, ci_blocks
 };
 
 // Wavefronts per workgroup: (g block, x block) pairs x parts of a stage's pixels. Blocks of 64 x 64 and those of a
@@ -175,9 +177,8 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
   // Workgroups are dealt to the 8 XCDs round robin; the ranges are numbered so that one
   // XCD holds neighbouring column strips, whose x rows share cache lines in that XCD's L2.
   const unsigned wg_rank = gridDim.x % 8 == 0 ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
-  const long long per = (p.total_stages + gridDim.x - 1) / gridDim.x;
-  const long long s_begin = min(per * wg_rank, p.total_stages);
-  const long long s_end = min(per * (wg_rank + 1), p.total_stages);
+  const long long s_begin = min(p.per * wg_rank, p.total_stages);
+  const long long s_end = min(p.per * (wg_rank + 1), p.total_stages);
 
   // ---- the block of channels
   constexpr int KD = CXB == 3 ? 3 : 1, CIN_B = XC / KD;  // three x blocks are the depth taps of 32 channels
@@ -186,8 +187,8 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
   const int block = blockIdx.y;
   bool first_x;
   {
-    const int pair_k = block % p.npairs, rest = block / p.npairs;
-    const int ci0 = (rest % p.ci_blocks) * CIN_B, co0 = (rest / p.ci_blocks) * GC;
+    const int rest = jg::quotient(block, p.by_pairs), pair_k = block - rest * p.npairs, co_block = jg::quotient(rest, p.by_ci);
+    const int ci0 = (rest - co_block * p.ci_blocks) * CIN_B, co0 = co_block * GC;
     const int gpart = (int)((p.gparts >> (2 * pair_k)) & 3u), xpart = (int)((p.xparts >> (2 * pair_k)) & 3u);
     cin_valid = min(CIN_B, p.cin - ci0);
     cout_valid = min(GC, p.cout - co0);
@@ -290,6 +291,14 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
   };
   auto decode = [&](long long stage) {
     Cursor c;
+    if (p.total_stages < (1ll << 31)) {
+      const int col = jg::quotient((uint32_t)stage, p.by_rp), plane = jg::quotient(col, p.by_ct);
+      c.hp = (int)stage - col * p.row_pairs;
+      c.ct = col - plane * p.col_tiles;
+      c.n = jg::quotient(plane, p.by_od);
+      c.od = plane - c.n * p.Dout;
+      return c;
+    }
     c.hp = (int)(stage % p.row_pairs);
     long long t = stage / p.row_pairs;
     c.ct = (int)(t % p.col_tiles);
@@ -1116,6 +1125,12 @@ int mfma_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom
   p.row_pairs = (g.out[1] + SR - 1) / SR;
   p.col_tiles = (g.out[2] + stage_columns(g) - 1) / stage_columns(g);
   p.total_stages = stage_count(g);
+  p.per = (p.total_stages + plan.wgs - 1) / plan.wgs;
+  p.by_rp = jg::div_by(p.row_pairs);
+  p.by_ct = jg::div_by(p.col_tiles);
+  p.by_od = jg::div_by(p.Dout);
+  p.by_pairs = jg::div_by(p.npairs);
+  p.by_ci = jg::div_by(p.ci_blocks);
   // Every stage whole and every window inside x: the kernel without the border path (see ALLIN).
   constexpr int SW = Stage<1>::SW;
   const bool all_inside = g.s[2] == 1 && even == 1 && xt == nullptr && g.p[0] == 0 && g.p[1] == 0 && g.p[2] == 0 &&

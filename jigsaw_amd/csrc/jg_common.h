@@ -56,6 +56,20 @@ __host__ __device__ static inline uint16_t f32_to_bf16(float f) {
   return (uint16_t)(r >> 16);
 }
 
+// Division by a number that holds for a whole launch, of numbers below 2^31: m = 2^(32 + s) / d rounded up, s < 0 for d = 1. A division of
+// the compiler's own is 30 instructions and more, over 100 in 64 bits, and a tile's place takes half a dozen of them.
+struct Div {
+  uint32_t m;
+  int s;
+};
+inline Div div_by(int d) {
+  if (d <= 1) return {0u, -1};
+  int bits = 0;
+  while ((1ll << bits) < d) ++bits;
+  return {(uint32_t)(((1ull << (31 + bits)) + d - 1) / d), bits - 1};
+}
+__device__ __forceinline__ uint32_t quotient(uint32_t n, const Div& d) { return d.s < 0 ? n : __umulhi(n, d.m) >> d.s; }
+
 static inline int cdiv(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
 // Compute units of the device (of a partition of it, where the device is one): what the host-side rules that fill the

@@ -38,19 +38,9 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-// Division by a number that holds for a whole launch, of numbers below 2^31: m = 2^(32 + s) / d rounded up, s < 0 for d = 1. A division of
-// the compiler's own is 30 instructions and more, over 100 in 64 bits, and the offsets of a tile take a dozen (see proj_nt_kernel).
-struct Div {
-  uint32_t m;
-  int s;
-};
-Div div_by(int d) {
-  if (d <= 1) return {0u, -1};
-  int bits = 0;
-  while ((1ll << bits) < d) ++bits;
-  return {(uint32_t)(((1ull << (31 + bits)) + d - 1) / d), bits - 1};
-}
-__device__ __forceinline__ uint32_t quotient(uint32_t n, const Div& d) { return d.s < 0 ? n : __umulhi(n, d.m) >> d.s; }
+using jg::Div;
+using jg::div_by;
+using jg::quotient;
 
 struct Map {
   int heads;     // 0: row-major with leading dimension ld; 1: (t, B, H, S, D)
