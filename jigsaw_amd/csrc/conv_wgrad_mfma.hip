@@ -38,6 +38,7 @@
 //   Reduction   the parts of a pair are added in LDS, the workgroup's partial goes
 //               to the workspace; a second kernel sums the partials in a fixed order
 //               (deterministic) and writes gw in the weight layout and gb, in their own dtype.
+#include <algorithm>
 #include <cmath>
 
 #include "conv_common.h"
@@ -111,6 +112,13 @@ constexpr int wgrad_parts(int cgb, int cxb) { return cgb * cxb <= 2 ? 4 : 2; }
 constexpr int wgrad_threads(int cgb, int cxb) {
   const int waves = cgb * cxb * wgrad_parts(cgb, cxb);
   return waves > 4 ? 512 : 64 * waves;
+}
+// LDS of a workgroup: two buffers of g and the ring of x, in whose place the parts meet at the end.
+template <int CGB, int CXB, int ST>
+constexpr size_t wgrad_lds() {
+  const size_t stage = 2 * (size_t)(32 * CGB * Stage<ST>::G_CH) + (size_t)(32 * CXB * Stage<ST>::X_CH);
+  const size_t waves = CGB * CXB * wgrad_parts(CGB, CXB), meet = waves * (12 - 12 / wgrad_parts(CGB, CXB)) * 1024;
+  return stage > meet ? stage : meet;
 }
 // Workgroups of one pair fit a compute unit twice.
 constexpr int wgrad_waves_per_simd(int cgb, int cxb) { return wgrad_parts(cgb, cxb) == 4 || wgrad_threads(cgb, cxb) == 512 ? 2 : 1; }
@@ -777,42 +785,46 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
     }
   }
 
-  // Partial of this workgroup. The parts of a pair meet in LDS first (the stage buffers are free: a barrier closed the last
-  // stage), three taps at a time, the upper half of them with the lower and so on, which leaves one of them to go to memory and
-  // come back. A lane's 16 values of a tap leave as four 16-byte pieces, [tap9][pair][4][lane][4].
-  static_assert(CGB * CXB * (PARTS / 2) * 3 * 4096 <= 2 * G_BYTES + XC * X_CH, "three taps of half of the parts fit the stage buffers");
+  // Partial of this workgroup. The parts of a pair meet in LDS (the stage buffers are free: a barrier closed the last stage), three taps
+  // at a time: their twelve 16-byte pieces a lane are dealt to the parts, a part leaves the others' with them, adds up its own and
+  // stores them, [tap9][pair][4][lane][4]. (Upper parts handing all of theirs to the lower ones, half of them at a time, kept most
+  // wavefronts waiting at twelve barriers: 3.4 us of a 64 x 32 block, 3.1 of 32 x 32, where this takes 2.8 and 2.3.)
+  constexpr int OWN = 12 / PARTS;  // pieces of three taps that a part adds up
+  static_assert(CWAVES * (12 - OWN) * 1024 <= wgrad_lds<CGB, CXB, ST>(), "the pieces of three taps fit");
   float* const out = p.part + slot * (size_t)(9 * GC * XC) + pair * 1024 + lane * 4;
 #pragma unroll
-  for (int kh = 0; kh < 3; ++kh)
+  for (int kh = 0; kh < 3; ++kh) {
+    // [pair][part that owns][part that gives, without the owner][piece][lane][4]
+    auto place = [&](int owner, int giver, int k) {
+      return reinterpret_cast<float*>(smem) + (((pair * PARTS + owner) * (PARTS - 1) + (giver < owner ? giver : giver - 1)) * OWN + k) * 256 + lane * 4;
+    };
+    auto piece = [&](int q) { return f32x4{acc[kh][q / 4][4 * (q % 4)], acc[kh][q / 4][4 * (q % 4) + 1], acc[kh][q / 4][4 * (q % 4) + 2], acc[kh][q / 4][4 * (q % 4) + 3]}; };
+    if (wave < CWAVES) {
 #pragma unroll
-    for (int step = PARTS / 2; step > 0; step /= 2) {
-      float* const meet = reinterpret_cast<float*>(smem) + (pair * (PARTS / 2) + part % step) * 3 * 1024 + lane * 4;
-      if (wave < CWAVES && part >= step && part < 2 * step) {
+      for (int owner = 0; owner < PARTS; ++owner)
+        if (owner != part) {
 #pragma unroll
-        for (int kw = 0; kw < 3; ++kw)
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            *reinterpret_cast<f32x4*>(meet + kw * 1024 + j * 256) =
-                f32x4{acc[kh][kw][4 * j], acc[kh][kw][4 * j + 1], acc[kh][kw][4 * j + 2], acc[kh][kw][4 * j + 3]};
-      }
-      __syncthreads();
-      if (wave < CWAVES && part < step) {
-#pragma unroll
-        for (int kw = 0; kw < 3; ++kw)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            f32x4 v = *reinterpret_cast<const f32x4*>(meet + kw * 1024 + j * 256);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] += acc[kh][kw][4 * j + k];
-            if (step == 1)
-              *reinterpret_cast<f32x4*>(out + (size_t)(kh * 3 + kw) * (GC * XC) + j * 256) = v;
-            else
-#pragma unroll
-              for (int k = 0; k < 4; ++k) acc[kh][kw][4 * j + k] = v[k];
-          }
-      }
-      __syncthreads();
+          for (int k = 0; k < OWN; ++k) *reinterpret_cast<f32x4*>(place(owner, part, k)) = piece(owner * OWN + k);
+        }
     }
+    __syncthreads();
+    if (wave < CWAVES) {
+#pragma unroll
+      for (int owner = 0; owner < PARTS; ++owner)
+        if (owner == part) {
+#pragma unroll
+          for (int k = 0; k < OWN; ++k) {
+            f32x4 v[PARTS];
+#pragma unroll
+            for (int g = 0; g < PARTS; ++g) v[g] = g == owner ? piece(owner * OWN + k) : *reinterpret_cast<const f32x4*>(place(owner, g, k));
+            const int q = owner * OWN + k;
+            const f32x4 sum = PARTS == 4 ? (v[0] + v[2]) + (v[1] + v[3]) : v[0] + v[1];
+            *reinterpret_cast<f32x4*>(out + (size_t)(kh * 3 + q / 4) * (GC * XC) + q % 4 * 256) = sum;
+          }
+        }
+    }
+    __syncthreads();
+  }
 }
 
 // gw = sum over the partials of a block of channels (its workgroups, and in split mode its part pairs, which
@@ -983,6 +995,11 @@ Plan plan_of(const ConvGeom& g, int parts) {
   if (n >= 8) n = n / 8 * 8;
   if (n > stages) n = stages;
   if (n < 1) n = 1;
+  // No more than the walks need: 1080 stages in walks of four are 270 workgroups, of 336 that the rule asks for 66 wrote
+  // a partial of nothing.
+  const long long walk = (stages + n - 1) / n, busy = (stages + walk - 1) / walk;
+  if (n >= 8) n = std::min(n, (busy + 7) / 8 * 8);
+  else n = busy;
   p.wgs = (int)n;
   return p;
 }
@@ -990,8 +1007,7 @@ Plan plan_of(const ConvGeom& g, int parts) {
 template <int CGB, int CXB>
 int launch(const WgradParams& p, int even, bool f16, bool all_inside, int stride, dim3 grid, hipStream_t s, const char* who) {
   constexpr int THREADS = wgrad_threads(CGB, CXB);
-  const size_t lds = stride == 2 ? 2 * (size_t)(32 * CGB * Stage<2>::G_CH) + (size_t)(32 * CXB * Stage<2>::X_CH)
-                                 : 2 * (size_t)(32 * CGB * Stage<1>::G_CH) + (size_t)(32 * CXB * Stage<1>::X_CH);
+  const size_t lds = stride == 2 ? wgrad_lds<CGB, CXB, 2>() : wgrad_lds<CGB, CXB, 1>();
   void (*kern)(WgradParams) = nullptr;
   if (stride == 2) {
     if constexpr (CXB != 3) {
