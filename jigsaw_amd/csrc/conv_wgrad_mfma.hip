@@ -40,6 +40,7 @@
 //               (deterministic) and writes gw in the weight layout and gb, in their own dtype.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "conv_common.h"
 
@@ -828,11 +829,12 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
 }
 
 // gw = sum over the partials of a block of channels (its workgroups, and in split mode its part pairs, which
-// lie behind each other), and gb the same over the bias partials. A workgroup owns one run of 256 values of a
-// block's partial (a tap, a pair, four registers), a lane four of them; its 8 wavefronts take every eighth
-// partial in chains of their own and the sums are added in a fixed order (deterministic). What bounds it is
-// the latency of the chains: 16-byte loads, eight in flight per lane.
-// The workgroups behind those of the last block add up bias partials, one lane per channel.
+// lie behind each other), and gb the same over the bias partials. A workgroup owns a run of 256 / SUB values of a
+// block's partial (a tap, a pair, four registers and 64 / SUB lanes of the kernel above), a lane four of them; its 8 wavefronts
+// take 8 SUB partials at a time in chains of their own and the sums are added in a fixed order (deterministic). What bounds it is
+// the latency of the chains, 16-byte loads, eight in flight a lane: a block of 32 x 32 is 36 runs of 256 values, which left most of
+// the chip idle (reduce_subs; RED_FIGURES).
+// The workgroups behind those of the last block add up bias partials, 16 channels each, four partials a wavefront at a time.
 struct ReduceParams {
   const float* part;
   const float* bias_part;
@@ -844,20 +846,22 @@ struct ReduceParams {
   int gw_blocks;              // workgroups that reduce gw
   int bias_cout, bias_parts;  // output channels, and parts of g whose bias sums belong together
 };
-constexpr int RED_WAVES = 8;
+constexpr int RED_WAVES = 8, BIAS_CHANNELS = 16;
 template <int OUT>  // dtype of gw and gb: 0 bf16, 1 fp32, 2 fp16
 __device__ __forceinline__ void store_gradient(void* out, size_t at, float v) {
   if (OUT == 1) static_cast<float*>(out)[at] = v;
   else if (OUT == 2) static_cast<_Float16*>(out)[at] = (_Float16)v;
   else static_cast<uint16_t*>(out)[at] = jg::f32_to_bf16(v);
 }
-template <int OUT>
+template <int OUT, int SUB>
 __global__ __launch_bounds__(64 * RED_WAVES) void wgrad_reduce_kernel(ReduceParams p) {
+  constexpr int LANES = 64 / SUB, CHAINS = RED_WAVES * SUB;  // lanes of a run, chains of a workgroup
   __shared__ f32x4 red[RED_WAVES][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if ((int)blockIdx.x >= p.gw_blocks) {
-    // bias: 64 channels per workgroup; a channel's block at x block 0 and x part 0 holds its sums
-    const int c = ((int)blockIdx.x - p.gw_blocks) * 64 + lane;
+    // bias: a channel's block at x block 0 and x part 0 holds its sums
+    const int c = ((int)blockIdx.x - p.gw_blocks) * BIAS_CHANNELS + lane % BIAS_CHANNELS, first = w * (64 / BIAS_CHANNELS) + lane / BIAS_CHANNELS;
+    constexpr int STEP = RED_WAVES * (64 / BIAS_CHANNELS);
     float s = 0.0f;
     if (c < p.bias_cout) {
       for (int gp = p.bias_parts - 1; gp >= 0; --gp) {
@@ -867,19 +871,21 @@ __global__ __launch_bounds__(64 * RED_WAVES) void wgrad_reduce_kernel(ReducePara
         const size_t slot0 = ((size_t)(row / p.GC) * p.ci_blocks * p.npairs + pair_k) * p.wgs;
         const float* src = p.bias_part + slot0 * p.GC + row % p.GC;
         float c8[8] = {};
-        for (int k = w; k < p.wgs; k += 8 * RED_WAVES) {
+        for (int k = first; k < p.wgs; k += 8 * STEP) {
 #pragma unroll
           for (int u = 0; u < 8; ++u) {
-            const int at = k + u * RED_WAVES;
+            const int at = k + u * STEP;
             c8[u] += at < p.wgs ? src[(size_t)at * p.GC] : 0.0f;
           }
         }
         s += ((c8[0] + c8[1]) + (c8[2] + c8[3])) + ((c8[4] + c8[5]) + (c8[6] + c8[7]));
       }
     }
+#pragma unroll
+    for (int o = BIAS_CHANNELS; o < 64; o <<= 1) s += __shfl_xor(s, o, 64);
     red[w][lane].x = s;
     __syncthreads();
-    if (w != 0 || c >= p.bias_cout) return;
+    if (w != 0 || lane >= BIAS_CHANNELS || c >= p.bias_cout) return;
     s = 0.0f;
 #pragma unroll
     for (int k = 0; k < RED_WAVES; ++k) s += red[k][lane].x;
@@ -887,33 +893,39 @@ __global__ __launch_bounds__(64 * RED_WAVES) void wgrad_reduce_kernel(ReducePara
     return;
   }
   const int runs = 9 * p.pairs * 4;  // runs of 256 values in a block's partial
-  const int blk = blockIdx.x / runs, run = blockIdx.x - blk * runs;
+  const int own = blockIdx.x / SUB, blk = own / runs, run = own - blk * runs;
+  const int at = (int)(blockIdx.x % SUB) * LANES + lane % LANES;  // the lane of the kernel above whose values these are
   const int slots = p.wgs * p.npairs;
   const size_t stride = (size_t)runs * 256;
-  const float* src = p.part + (size_t)blk * slots * stride + (size_t)run * 256 + lane * 4;
+  const float* src = p.part + (size_t)blk * slots * stride + (size_t)run * 256 + at * 4;
   f32x4 c[8] = {};
-  int k = w;
-  for (; k + 7 * RED_WAVES < slots; k += 8 * RED_WAVES) {
+  int k = w * SUB + lane / LANES;
+  for (; k + 7 * CHAINS < slots; k += 8 * CHAINS) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) c[u] += *reinterpret_cast<const f32x4*>(src + (size_t)(k + u * RED_WAVES) * stride);
+    for (int u = 0; u < 8; ++u) c[u] += *reinterpret_cast<const f32x4*>(src + (size_t)(k + u * CHAINS) * stride);
   }
 #pragma unroll
   for (int u = 0; u < 7; ++u)
-    if (k + u * RED_WAVES < slots) c[u] += *reinterpret_cast<const f32x4*>(src + (size_t)(k + u * RED_WAVES) * stride);
-  red[w][lane] = ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
+    if (k + u * CHAINS < slots) c[u] += *reinterpret_cast<const f32x4*>(src + (size_t)(k + u * CHAINS) * stride);
+  f32x4 sum = ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
+#pragma unroll
+  for (int o = LANES; o < 64; o <<= 1)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) sum[u] += __shfl_xor(sum[u], o, 64);
+  red[w][lane] = sum;
   __syncthreads();
-  if (w != 0) return;
-  f32x4 sum = red[0][lane];
+  if (w != 0 || lane >= LANES) return;
+  sum = red[0][lane];
 #pragma unroll
   for (int u = 1; u < RED_WAVES; ++u) sum += red[u][lane];
   const int j = run & 3, pair = (run >> 2) % p.pairs, tap = (run >> 2) / p.pairs;
   const int cb = pair / p.CXB, ib = pair % p.CXB;
-  const int cx = ib * 32 + (lane & 31), kd = cx / p.cin_b;
+  const int cx = ib * 32 + (at & 31), kd = cx / p.cin_b;
   const int ci = (blk % p.ci_blocks) * p.cin_b + cx % p.cin_b;
   if (ci >= p.cin) return;
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    const int co = (blk / p.ci_blocks) * p.GC + cb * 32 + 8 * j + 4 * (lane >> 5) + u;
+    const int co = (blk / p.ci_blocks) * p.GC + cb * 32 + 8 * j + 4 * (at >> 5) + u;
     if (co < p.cout) store_gradient<OUT>(p.gw, (((size_t)co * p.cin + ci) * p.KD + kd) * 9 + tap, sum[u]);
   }
 }
@@ -1002,6 +1014,12 @@ Plan plan_of(const ConvGeom& g, int parts) {
   else n = busy;
   p.wgs = (int)n;
   return p;
+}
+
+// Pieces that a run of 256 values is cut into: up to two workgroups a compute unit.
+int reduce_subs(long long runs) {
+  const long long most = 2ll * jg::cu_count();
+  return 4 * runs <= most ? 4 : 2 * runs <= most ? 2 : 1;
 }
 
 template <int CGB, int CXB>
@@ -1175,10 +1193,19 @@ int mfma_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom
   r.KD = plan.KD; r.cin = p.cin; r.cout = p.cout; r.ci_blocks = plan.ci_blocks;
   r.bias_cout = g.cout; r.bias_parts = parts;
   r.gw_blocks = plan.co_blocks * plan.ci_blocks * 9 * r.pairs * 4;
-  const unsigned rgrid = (unsigned)r.gw_blocks + (gb != nullptr ? (unsigned)(g.cout + 63) / 64 : 0u);
-  if (dtype == JG_F32) wgrad_reduce_kernel<1><<<rgrid, 64 * RED_WAVES, 0, s>>>(r);
-  else if (f16) wgrad_reduce_kernel<2><<<rgrid, 64 * RED_WAVES, 0, s>>>(r);
-  else wgrad_reduce_kernel<0><<<rgrid, 64 * RED_WAVES, 0, s>>>(r);
+  const unsigned bgrid = gb != nullptr ? (unsigned)(g.cout + BIAS_CHANNELS - 1) / BIAS_CHANNELS : 0u;
+  auto reduce = [&](auto sub) {
+    constexpr int SUB = decltype(sub)::value;
+    r.gw_blocks *= SUB;
+    const unsigned rgrid = (unsigned)r.gw_blocks + bgrid;
+    if (dtype == JG_F32) wgrad_reduce_kernel<1, SUB><<<rgrid, 64 * RED_WAVES, 0, s>>>(r);
+    else if (f16) wgrad_reduce_kernel<2, SUB><<<rgrid, 64 * RED_WAVES, 0, s>>>(r);
+    else wgrad_reduce_kernel<0, SUB><<<rgrid, 64 * RED_WAVES, 0, s>>>(r);
+  };
+  const int subs = reduce_subs(r.gw_blocks);
+  if (subs == 4) reduce(std::integral_constant<int, 4>{});
+  else if (subs == 2) reduce(std::integral_constant<int, 2>{});
+  else reduce(std::integral_constant<int, 1>{});
   JG_CHECK_LAUNCH(who);
   if (plan.parts_in_block > 1) {
     // few channels: all part products came from one block (the parts are channels of it); the ones that count
