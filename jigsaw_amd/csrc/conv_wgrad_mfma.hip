@@ -213,8 +213,11 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
   // ---- per-thread chunk bookkeeping, fixed for the whole kernel. Chunk q < G_CHUNKS
   // is 8 pixels of a g row, the others 8 pixels of one of the two x rows of a pair.
   uint32_t c_goff[ROUNDS];  // byte offset from the origin of its tensor window
-  uint32_t c_lds[ROUNDS];   // byte offset inside the g buffer / inside the x ring, row slot 0
-  uint32_t x_row = 0;       // two bits per round: the chunk's row among the new ones
+  // byte offset inside the g buffer / inside the x ring, row slot 0 (stride 1: of the chunk's own row, the new rows being a pair that
+  // never lies across the ring's end)
+  uint32_t c_lds[ROUNDS];
+  uint32_t x_row = 0;       // stride 2, two bits per round: the chunk's row among the new ones
+  static_assert(ST == 2 || RING % NEW == 0, "pairs of rows stay together in the ring");
 #pragma unroll
   for (int rd = 0; rd < ROUNDS; ++rd) {
     const int q = tid + rd * THREADS;
@@ -231,8 +234,8 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
       const int kd = ch / CIN_B, cib = ch - kd * CIN_B;
       const int ci = cib < cin_valid ? cib : cin_valid - 1;
       c_goff[rd] = (uint32_t)((ci * x_cs + kd * plane_x + (size_t)r2 * p.Win + c8 * 8) * 2);
-      c_lds[rd] = (uint32_t)(ch * X_CH + c8 * (16 / ST));
-      x_row |= (uint32_t)r2 << (2 * rd);
+      c_lds[rd] = (uint32_t)(ch * X_CH + c8 * (16 / ST) + (ST == 1 ? r2 * X_ROW : 0));
+      if (ST == 2) x_row |= (uint32_t)r2 << (2 * rd);
     } else {
       c_goff[rd] = 0;
       c_lds[rd] = 0;
@@ -248,7 +251,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
     const int kd = ch / CIN_B, cib = ch - kd * CIN_B;
     const int ci = cib < cin_valid ? cib : cin_valid - 1;
     t_goff = (uint32_t)((ci * x_cs + kd * plane_x + (size_t)r2 * p.Win + 64) * 2);
-    t_lds = (uint32_t)(ch * X_CH + 128 / ST);
+    t_lds = (uint32_t)(ch * X_CH + 128 / ST + (ST == 1 ? r2 * X_ROW : 0));
   }
   // the same x offsets inside the own tile (framed input)
   const size_t plane_t = (size_t)p.tn_h * p.tn_w, t_cs = plane_t * p.tn_d;
@@ -293,10 +296,21 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
 
   // Loads of one stage into `v`: its two g rows (want_g) and one pair of its x rows
   // (pair 0: the rows shared with the stage above, pair 1: the two new rows).
-  // Position of a stage: row pair (fastest), column tile, output depth, batch entry.
-  // Decoded once with divisions, then stepped, so the stage loop has none.
+  // Position of a stage: row pair (fastest), column tile, output depth, batch entry, and the first bytes of its g rows and its new x
+  // rows. Decoded once, then stepped: down a strip the two addresses move by a constant, and only a new strip works
+  // them out. (From scratch in every stage they were most of its 116 scalar instructions, whose issue no matrix instruction of the
+  // SIMD's other wavefront hides: SCALAR_FIGURES.)
   struct Cursor {
     int hp, ct, od, n;
+    const char *g, *x;
+  };
+  const uint32_t g_step = 2u * SR * (uint32_t)p.Wout, x_step = 2u * NEW * (uint32_t)p.Win;  // of one stage
+  auto place = [&](Cursor& c) {
+    c.g = reinterpret_cast<const char*>(gb) +
+          2 * (((size_t)c.n * p.cout_total * p.Dout + c.od) * plane_g + (size_t)(c.hp * SR) * p.Wout + c.ct * SW);
+    c.x = reinterpret_cast<const char*>(xb) +
+          2 * ((ptrdiff_t)((size_t)c.n * p.cin_total * p.Din * plane_x) + (ptrdiff_t)(c.od - p.pad_d) * (ptrdiff_t)plane_x +
+               (ptrdiff_t)(ST * c.hp * SR - p.pad_h + XR - NEW) * p.Win + (ST * c.ct * SW - p.pad_w - LEAD));
   };
   auto decode = [&](long long stage) {
     Cursor c;
@@ -306,17 +320,20 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
       c.ct = col - plane * p.col_tiles;
       c.n = jg::quotient(plane, p.by_od);
       c.od = plane - c.n * p.Dout;
-      return c;
+    } else {
+      c.hp = (int)(stage % p.row_pairs);
+      long long t = stage / p.row_pairs;
+      c.ct = (int)(t % p.col_tiles);
+      t /= p.col_tiles;
+      c.od = (int)(t % p.Dout);
+      c.n = (int)(t / p.Dout);
     }
-    c.hp = (int)(stage % p.row_pairs);
-    long long t = stage / p.row_pairs;
-    c.ct = (int)(t % p.col_tiles);
-    t /= p.col_tiles;
-    c.od = (int)(t % p.Dout);
-    c.n = (int)(t / p.Dout);
+    place(c);
     return c;
   };
   auto advance = [&](Cursor& c) {
+    c.g += g_step;
+    c.x += x_step;
     if (++c.hp == p.row_pairs) {
       c.hp = 0;
       if (++c.ct == p.col_tiles) {
@@ -326,6 +343,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
           ++c.n;
         }
       }
+      place(c);
     }
   };
 
@@ -335,11 +353,8 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
     const int oh0 = hp * SR, ow0 = ct * SW;
     // first of the rows: of the new ones, or (xpair 0) as many rows further up, the last of which a first stage lacks
     const int id0 = od - p.pad_d, ih0 = ST * oh0 - p.pad_h + XR - (xpair ? 1 : 2) * NEW, iw0 = ST * ow0 - p.pad_w - LEAD;
-    const char* g_org = reinterpret_cast<const char*>(gb) +
-                        2 * (((size_t)n * p.cout_total * p.Dout + od) * plane_g + (size_t)oh0 * p.Wout + ow0);
-    const char* x_org = reinterpret_cast<const char*>(xb) +
-                        2 * ((ptrdiff_t)((size_t)n * p.cin_total * p.Din * plane_x) + (ptrdiff_t)id0 * (ptrdiff_t)plane_x +
-                             (ptrdiff_t)ih0 * p.Win + iw0);
+    const char* const g_org = cur.g;
+    const char* const x_org = xpair ? cur.x : cur.x - x_step;
     // (with LEAD the window's last dword holds one pixel more than is used; it shares its dword with one that is)
     const bool rows_inside = oh0 + SR <= p.Hout && ih0 >= 0 && ih0 + NEW <= p.Hin && id0 >= 0 && id0 + KD <= p.Din;
     // All that a stage's loads of x and g reach lies inside the tensors, whatever columns the rows have
@@ -574,8 +589,11 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
         if (G_CHUNKS % THREADS == 0 || q < G_CHUNKS) *reinterpret_cast<u32x4*>(smem + gbuf * G_BYTES + c_lds[rd]) = val;
         if (bias_part != nullptr) bsum[rd] += counted ? sum_of_8<F16>(val) : 0.0f;
       } else if (q < CHUNKS) {
-        int slot = slot0 + (int)((x_row >> (2 * rd)) & 3u);
-        if (slot >= RING) slot -= RING;
+        int slot = slot0;
+        if (ST == 2) {
+          slot += (int)((x_row >> (2 * rd)) & 3u);
+          if (slot >= RING) slot -= RING;
+        }
         unsigned char* const at = lds_x + c_lds[rd] + slot * X_ROW;
         if (ST == 1) {
           *reinterpret_cast<u32x4*>(at) = val;
@@ -588,8 +606,11 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
       }
     }
     if (has_tail) {
-      int slot = slot0 + tid % NEW;
-      if (slot >= RING) slot -= RING;
+      int slot = slot0;
+      if (ST == 2) {
+        slot += tid % NEW;
+        if (slot >= RING) slot -= RING;
+      }
       unsigned char* at = lds_x + t_lds + slot * X_ROW;
       uint32_t t = sg.tail, tb = sg.tail_b;
       if (EVEN == 0) t = __builtin_amdgcn_alignbit(tb, t, (sg.odd >> 31) << 4);
@@ -631,8 +652,10 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
     for (int r = 0; r < PR; ++r) f.a[r] = *reinterpret_cast<const u32x4*>(gb + (row0 + r) * (SW * 2) + cg * 32);
 #pragma unroll
     for (int rho = 0; rho < PXR; ++rho) {
-      int slot = base + ST * row0 + rho;
+      // (stride 1: two pairs of rows, each in one piece of the ring)
+      int slot = base + ST * row0 + (ST == 1 ? rho / NEW * NEW : rho);
       if (slot >= RING) slot -= RING;
+      if (ST == 1) slot += rho % NEW;
       f.d[rho] = *reinterpret_cast<const u32x4*>(xb + slot * X_ROW + cg * 32);
       f.d4[rho] = *reinterpret_cast<const uint32_t*>(xb + slot * X_ROW + cg * 32 + 16);
       f.d5[rho] = 0u;
@@ -711,7 +734,8 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
       // the compiler then waits for the loads at the end of the stage that issued them (to copy
       // the registers together) instead of where they are stored, half a stage later.
       if (s_begin + 1 < s_end) advance(c_next);
-      Cursor c_store = c_next;          // stage whose registers are stored next (st + 1)
+      Cursor c_store = c_next;  // stage whose registers are stored next
+      const int stages = (int)(s_end - s_begin);
       issue_loads(stg, c_next, true, 1);
       if (s_begin + 2 < s_end) advance(c_next);
       __syncthreads();
@@ -730,11 +754,11 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
       // every stage what the tensor's ends cost): 1 x 30 -> 9 of 38 x 66 x 15 45.1 -> 40.7 us, 2 x 64 -> 64 of 30 x 50 x 20 79.6 -> 74.1,
       // 2 x 48 -> 8 of 36 x 48 x 76 83.5 -> 80.0.
       constexpr bool kBothFirst = CWAVES == 8 || ALLIN || FRAMED;
-      for (long long st = s_begin; st < s_end; ++st) {
+      for (int st = 0; st < stages; ++st) {
         Frags f0, f1;
         (void)f1;
         if (stage_first) {
-          store_loads(stg, true, gbuf ^ 1, wrap(base + XR), st + 1 < s_end);
+          store_loads(stg, true, gbuf ^ 1, wrap(base + XR), st + 1 < stages);
           issue_loads(stg, c_next, true, 1);
         }
         if (wave < CWAVES) {
@@ -744,16 +768,17 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
           if (GROUPS == 2 && CWAVES == 8) mfma_group(f1);
         }
         if (!stage_first) {
-          store_loads(stg, true, gbuf ^ 1, wrap(base + XR), st + 1 < s_end);
+          store_loads(stg, true, gbuf ^ 1, wrap(base + XR), st + 1 < stages);
           issue_loads(stg, c_next, true, 1);
         }
         if (GROUPS == 2 && CWAVES != 8 && wave < CWAVES) {
           if (!kBothFirst) read_group(f1, gbuf, base, 1);
           mfma_group(f1);
         }
-        if (st + 3 < s_end) advance(c_next);
+        const Cursor c_issued = c_next;
+        if (st + 3 < stages) advance(c_next);
         __syncthreads();
-        if (st + 1 < s_end && c_store.hp == 0) {
+        if (st + 1 < stages && c_store.hp == 0) {
           // the next stage starts a new strip: its first two x rows, on the spot
           Staged top;
           issue_loads(top, c_store, false, 0);
@@ -764,7 +789,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
           __builtin_amdgcn_s_waitcnt(0x0F70);
           __syncthreads();
         }
-        advance(c_store);
+        c_store = c_issued;
         base = wrap(base + NEW);
         gbuf ^= 1;
       }
