@@ -98,7 +98,7 @@ struct TileWalk {
 struct FwdParams {
   const uint16_t* x;    // (N, C, Din, Hin, Win) bf16: the tensor that is convolved
   const char* x_end;    // one past the last byte of x
-  const u32x4* wprep;   // prepared weights, [m_tile][group][tap9][wc16][kg][MT][8]
+  const u32x4* wprep;   // prepared weights, [m_tile][group][wc16][kg][tap9][MT][8]
   const uint16_t* wraw;  // the weights as they are, which each workgroup puts in order itself (arrange_weights); NULL: wprep
   int transposed;        // (with wraw) as in prep_weights_kernel
   const uint16_t* bias; // (M,) or NULL
@@ -170,7 +170,7 @@ __device__ __forceinline__ TileWalk walk_of() {
 }
 
 // ---------------------------------------------------------------- weight prep
-// dst[(((mt*ngroups + group)*9 + tap9)*wc16 + c16 in group)*2 + kg][m_local][8 k] (bf16), contraction channel
+// dst[(((mt*ngroups + group)*wc16 + c16 in group)*2 + kg)*9 + tap9][m_local][8 k] (bf16), contraction channel
 // k = kd*Cp + c (channels C..Cp-1 are zero padding). transposed = 0: A[m][k] = w[m][c][kd][kh][kw] (forward, w is
 // (M, C, KD, 3, 3)); transposed = 1: A[m][k] = w[c][m][KD-1-kd][2-kh][2-kw] (input
 // gradient, w is (C, M, KD, 3, 3)); transposed = 2: the six taps of a phase row of the strided input gradient
@@ -191,9 +191,9 @@ __global__ __launch_bounds__(256) void prep_weights_kernel(uint16_t* __restrict_
     int e = i & 7;
     int r = i >> 3;
     int ml = r % MT; r /= MT;
+    int tap = r % taps; r /= taps;
     int kg = r & 1; r >>= 1;
     int c16l = r % wc16; r /= wc16;
-    int tap = r % taps; r /= taps;
     int grp = r % ngroups;
     int mt = r / ngroups;
     const int m = (transposed == 2 ? mt >> 1 : mt) * MT + ml;
@@ -296,9 +296,9 @@ __global__ __launch_bounds__(256) void prep_weights_split_kernel(uint16_t* __res
     int e = i & 7;
     int r = i >> 3;
     int ml = r % MT; r /= MT;
+    int tap = r % taps; r /= taps;
     int kg = r & 1; r >>= 1;
     int c16l = r % wc16; r /= wc16;
-    int tap = r % taps; r /= taps;
     int grp = r % ngroups;
     int mt = r / ngroups;
     const int m = (transposed == 2 ? mt >> 1 : mt) * MT + ml;
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   float* lds_bias = reinterpret_cast<float*>(lds_in + 2 * STAGE_SLOTS);
 
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (scalar: what follows from it branches without masks)
   const int ln = lane & 31, kg = lane >> 5;
   // Wavefronts w and w + 4 share a SIMD. They hold different column halves, so when a tile's second
   // half lies past the row end every SIMD drops half of that tile's MFMAs, and row groups two apart,
@@ -496,7 +496,7 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
 #pragma unroll
       for (int t = 0; t < WTAPS; ++t) {
         const int tap = MODE != STRIDED_DGRAD && p.transposed ? TAPS - 1 - t : t;
-        lds_w[((size_t)tap * octs + o) * MT + m] = v[t];
+        lds_w[(o * WTAPS + tap) * MT + m] = v[t];
       }
     }
     __syncthreads();
@@ -561,19 +561,33 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   // the cursor enters a tile; inside a tile the step moves by additions.
   struct Cursor {
     int ti;          // index into this workgroup's tiles
-    int blk, inner;  // contraction block, channel offset inside it (= kd * Cp + c0)
+    int blk;         // contraction block
     int kd, c0;      // depth tap and first channel of the step
     int od;          // produced depth plane of the tile
     int ih0, iw0;    // window origin in the input plane
     bool window_in;  // rows and columns of the window lie inside the plane
     bool window_in_t;  // ... inside the rank's own tile (framed input)
+    bool depth_ok;   // the depth tap's plane exists
     const char* base;    // window origin in channel 0 of the batch entry, depth plane 0
     const char* base_t;  // the same in the rank's own tile (framed input)
+    const char* at;      // window origin in the step's first channel and plane (before the tensor where padded)
   } cur;
-  const int per_blk_ch = (p.nc16 / p.nblk) * CK;  // contraction channels (x depth taps) of one block
+  const uint32_t step_b = CK * chan_b;  // bytes between the steps of a depth tap
+  // The origin is worked out for a depth tap and moves by additions inside it. From scratch in every stage, with 64-bit products and
+  // comparisons, 64-bit lane addresses for each load, a product for each weight fragment's place and execution masks around what a whole
+  // wavefront skips, a stage had 160 scalar and 140 vector instructions beside 36 or 72 matrix instructions, which the SIMD's other wavefront
+  // hides only in part. Forward / gradient with the fold: 2 x 32 -> 32 of 128^3 285 -> 272 us / 387 -> 356, 2 x 48 -> 19 of
+  // 121 x 126 x 78 365 -> 350 / 454 -> 429, 1 x 54 -> 84 of 105 x 65 19.3 -> 17.5 / 24.5 -> 22.5, 4 x 64 -> 128 of 256^2 at stride 2 30.5 -> 28.7
+  // / 35.5 -> 32.9; 8 x 64 -> 64 of 1024^2 665 -> 667 / 792 -> 782 (matrix instructions and the fragments' reads).
+  auto cursor_tap = [&]() __attribute__((always_inline)) {
+    const int id = cur.od + cur.kd - p.pad_d;
+    cur.c0 = 0;
+    cur.depth_ok = id >= 0 && id < p.Din;
+    cur.at = cur.base + 2 * ((ptrdiff_t)((size_t)((int)((p.xmap >> (2 * cur.blk)) & 3u) * p.C) * chan_stride) + (ptrdiff_t)id * (ptrdiff_t)plane);
+  };
   auto cursor_enter = [&](int ti) __attribute__((always_inline)) {
     cur.ti = ti;
-    cur.blk = 0; cur.inner = 0; cur.kd = 0; cur.c0 = 0;
+    cur.blk = 0; cur.kd = 0; cur.c0 = 0;
     if (ti >= my_tiles) return;
     const TileCoord tc = coord(tile_of(ti));
     cur.od = tc.od;
@@ -588,42 +602,39 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
       cur.base_t = reinterpret_cast<const char*>(p.xt) +
                    2 * ((ptrdiff_t)((size_t)tc.n * p.Cx * chan_stride_t) + (ptrdiff_t)ht * p.tn_w + wt);
     }
+    cursor_tap();
   };
   auto cursor_advance = [&]() __attribute__((always_inline)) {
-    cur.inner += CK;
     cur.c0 += CK;
-    if (cur.c0 >= p.Cp) {
-      cur.c0 = 0;
-      ++cur.kd;
+    cur.at += step_b;
+    if (cur.c0 < p.Cp) return;
+    if (++cur.kd == p.KD) {
+      cur.kd = 0;
+      if (++cur.blk == p.nblk) {
+        cursor_enter(cur.ti + 1);
+        return;
+      }
     }
-    if (cur.inner == per_blk_ch) {
-      cur.inner = 0; cur.kd = 0; cur.c0 = 0;
-      if (++cur.blk == p.nblk) cursor_enter(cur.ti + 1);
-    }
+    cursor_tap();
   };
 
   // Loads of the stage under the cursor.
   auto issue_loads = [&]() __attribute__((always_inline)) {
-    const int kd = cur.kd, c0 = cur.c0;
-    const int cx0 = (int)((p.xmap >> (2 * cur.blk)) & 3u) * p.C + c0;  // first channel of the step in x
     // Channels of this task that exist (all 8 unless C is not a multiple of 16). The vector
     // path below reads the others anyway (they lie inside the tensor: the interior test covers
     // all 16 channel planes) and store_stage zeroes them; the guarded paths skip them.
-    stg_left = p.C - c0;
+    stg_left = p.C - cur.c0;
     const int cvalid = stg_left - g8 * 8;
-    const int id = cur.od + kd - p.pad_d;
-    const int ih0 = cur.ih0, iw0 = cur.iw0;
-    const bool depth_ok = id >= 0 && id < p.Din;
-    // wave-uniform origin of the stage window (lies before the tensor where padded)
-    const char* origin = cur.base + 2 * ((ptrdiff_t)((size_t)cx0 * chan_stride) + (ptrdiff_t)id * (ptrdiff_t)plane);
+    const char* const origin = cur.at;  // wave-uniform
     // The last octet of a row holds 2 pixels that are used and 6 that no fragment
     // reads, so it may run past the row end as long as it stays inside the tensor.
-    const char* last = origin + 2 * ((size_t)(CK - 1) * chan_stride + (size_t)(IN_ROWS - 1) * p.Win + OCTS * 8);
-    const bool interior = depth_ok && cur.window_in && last <= p.x_end;
+    const uint32_t span = (CK - 1) * chan_b + 2u * ((IN_ROWS - 1) * (uint32_t)p.Win + OCTS * 8);
+    const bool interior = cur.depth_ok && cur.window_in && __builtin_amdgcn_readfirstlane((int)((p.x_end - origin - span) >> 32)) >= 0;
     if (FRAMED) {
       // window inside the own tile (wave-uniform): read the tile itself, at whatever
       // alignment its rows give the window
-      const int dt = id - p.tlo_d;
+      const int dt = cur.od + cur.kd - p.pad_d - p.tlo_d;
+      const int cx0 = (int)((p.xmap >> (2 * cur.blk)) & 3u) * p.C + cur.c0;  // first channel of the step in x
       const char* origin_t = cur.base_t + 2 * ((ptrdiff_t)((size_t)cx0 * chan_stride_t) + (ptrdiff_t)dt * (ptrdiff_t)plane_t);
       if (dt >= 0 && dt < p.tn_d && cur.window_in_t) {
         stg_masked = false;
@@ -680,41 +691,52 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     // One set of loads for every window, from addresses that differ: a load under a condition leaves its register
     // with two possible values where the paths meet, and the compiler then waits for it right there, half a stage
     // before it is wanted (a border window took the whole latency of memory that way).
-    uintptr_t from = reinterpret_cast<uintptr_t>(origin);  // wave-uniform where the window lies inside the tensor
+    // A wave-uniform base and a 32-bit lane offset that walks the channels.
+    const char* from = origin;
     uint32_t off = t_off;
     uint32_t step = chan_b;
     int steps = 8;
     if (!interior) {
       // A window that sticks out of the tensor, or whose 16 channels do (a ragged last step). A task reads
       // its 16 bytes wherever they lie inside the tensor, also past the end of its row; store_stage clears
-      // the pixels that are not the row's. Tasks without any pixel of the tensor read the prepared weights
-      // instead, and so do those whose bytes reach over the tensor's own ends: store_stage fetches these.
-      const int ih = ih0 + t_row, iw = iw0 + t_col;
-      const bool row_ok = depth_ok && ih >= 0 && ih < p.Hin && cvalid > 0;
+      // the pixels that are not the row's. Tasks without any pixel of the tensor read the first bytes of the window instead (of the
+      // tensor, where the window starts outside of it; the prepared weights where there are no 16 bytes), and so do those whose bytes
+      // reach over the tensor's own ends: store_stage fetches these.
+      const int ih = cur.ih0 + t_row, iw = cur.iw0 + t_col;
+      const bool row_ok = cur.depth_ok && ih >= 0 && ih < p.Hin && cvalid > 0;
       const int first = max(0, min(8, -iw)), past = max(0, min(8, p.Win - iw));
       stg_mask = row_ok ? ((1u << past) - 1u) & ~((1u << first) - 1u) : 0u;
       // (not EVEN: the task before takes its last pixel from this one's first dword)
       const bool need = EVEN ? stg_mask != 0u : row_ok && iw - 1 < p.Win && iw + 8 > 0;
+      const char* const x0 = reinterpret_cast<const char*>(p.x);
       const char* a = origin + t_off;
-      const uint32_t span = (uint32_t)(min(cvalid, 8) - 1) * chan_b;
-      const bool fits = a >= reinterpret_cast<const char*>(p.x) && a + (size_t)span + 16 <= p.x_end;
+      const uint32_t span_here = (uint32_t)(min(cvalid, 8) - 1) * chan_b;
+      const bool fits = a >= x0 && a + (size_t)span_here + 16 <= p.x_end;
       if (need && !fits) stg_mask |= 0x100u;
-      from = reinterpret_cast<uintptr_t>(need && fits ? a : reinterpret_cast<const char*>(p.wprep));
+      if (origin < x0 || origin + 16 > p.x_end) from = x0 + 16 <= p.x_end ? x0 : reinterpret_cast<const char*>(p.wprep);
+      off = need && fits ? (uint32_t)(a - from) : 0u;
       step = need && fits ? chan_b : 0u;
       steps = cvalid;
-      off = 0;
     }
     if (!EVEN) {
-      off += (uint32_t)(from & 3);
-      from &= ~(uintptr_t)3;
-      stg_odd = 0;
+      off += (uint32_t)reinterpret_cast<uintptr_t>(from) & 3u;
+      from -= reinterpret_cast<uintptr_t>(from) & 3;
+      // every second channel starts on the other half of a dword where a channel has an odd number of pixels
+      stg_odd = ((off & 2u) != 0u ? 0xffu : 0u) ^ ((step & 2u) != 0u ? 0xaau : 0u);
+    }
+    uint32_t offs[8];
+    offs[0] = off;
+    if (stg_left >= CK) {  // wave-uniform: every channel of the step exists
+#pragma unroll
+      for (int c = 1; c < 8; ++c) offs[c] = offs[c - 1] + step;
+    } else {
+#pragma unroll
+      for (int c = 1; c < 8; ++c) offs[c] = offs[c - 1] + (c < steps ? step : 0u);
     }
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      const u32x4_a4 v = jg::load_16_bytes_at(from + (EVEN ? off : off & ~3u));
+      const u32x4_a4 v = jg::load_16_bytes_at(reinterpret_cast<uintptr_t>(from) + (EVEN ? offs[c] : offs[c] & ~3u));
       stg[c][0] = v.x; stg[c][1] = v.y; stg[c][2] = v.z; stg[c][3] = v.w;
-      if (!EVEN) stg_odd |= ((off >> 1) & 1u) << c;
-      off += c + 1 < steps ? step : 0u;
     }
   };
 
@@ -792,8 +814,8 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   u32x4 bnext;
   int a_step = -1;  // the step inside the weight group whose kw = 0 fragments `a` holds
   auto weight_frag = [&](int wstep, int kh, int kw, int cb) {
-    const u32x4* wt = lds_w + ((size_t)wstep * 2 + kg) * MT + ln;
-    return __builtin_bit_cast(bf16x8, wt[(size_t)(kh * KW + kw) * p.wc16 * 2 * MT + ch0 + cb * 32]);
+    const u32x4* wt = lds_w + kg * (WTAPS * MT) + ln + (wstep * (2 * WTAPS * MT) + ch0);  // a tap's distance is an immediate offset of the read
+    return __builtin_bit_cast(bf16x8, wt[(kh * KW + kw) * MT + cb * 32]);
   };
   auto compute_kw = [&](int buf, int wstep, int kw, int wstep_next) {  // wstep: the stage's step inside its weight group
     const u32x4* in = lds_in + buf * STAGE_SLOTS + kg * (IN_ROWS * ROW_SLOTS) + ST * wrow0 * ROW_SLOTS;
@@ -856,8 +878,8 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   auto compute_phases = [&](int buf, int wstep, int kw) __attribute__((always_inline)) {
     const bool upper = (blockIdx.y & 1) == 0;  // pa = 0: both row offsets have taps
     const u32x4* in = lds_in + buf * STAGE_SLOTS + kg * (IN_ROWS * ROW_SLOTS) + wrow0 * ROW_SLOTS + in_slot(wcol0 + ln + p.lead + kw);
-    const u32x4* wt = lds_w + ((size_t)wstep * 2 + kg) * MT + ln;
-    auto frag = [&](int tap) { return __builtin_bit_cast(bf16x8, wt[(size_t)tap * p.wc16 * 2 * MT]); };
+    const u32x4* wt = lds_w + kg * (WTAPS * MT) + ln + wstep * (2 * WTAPS * MT);
+    auto frag = [&](int tap) { return __builtin_bit_cast(bf16x8, wt[tap * MT]); };
     auto mfma = [&](const bf16x8& w, const bf16x8& b, f32x16& to) __attribute__((always_inline)) {
       to = F16 ? __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, b), to, 0, 0, 0)
                : __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, b, to, 0, 0, 0);
@@ -899,9 +921,9 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
     typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
     const int n = lane & 15, quad = (lane >> 4) & 1;  // pixel row / channel, half of the eight channels of a slot
     const u32x2* in = reinterpret_cast<const u32x2*>(lds_in + buf * STAGE_SLOTS + kg * (IN_ROWS * ROW_SLOTS) + n * ROW_SLOTS) + quad;
-    const u32x2* wt = reinterpret_cast<const u32x2*>(lds_w + ((size_t)wstep * 2 + kg) * MT + lch + n) + quad;
+    const u32x2* wt = reinterpret_cast<const u32x2*>(lds_w + kg * (WTAPS * MT) + n + (wstep * (2 * WTAPS * MT) + lch)) + quad;
     auto product = [&](int tap, int row, int col) __attribute__((always_inline)) {
-      const u32x2 a = wt[2 * (size_t)tap * p.wc16 * 2 * MT], b = in[2 * (row * ROW_SLOTS + in_slot(col))];
+      const u32x2 a = wt[2 * tap * MT], b = in[2 * (row * ROW_SLOTS + in_slot(col))];
       left = F16 ? __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), left, 0, 0, 0)
                  : __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), left, 0, 0, 0);
     };
@@ -927,10 +949,10 @@ __global__ __launch_bounds__(THREADS) void conv3x3_mfma_kernel(StripTable strips
   };
   auto compute_top = [&](int buf, int wstep) __attribute__((always_inline)) {
     const u32x4* in = lds_in + buf * STAGE_SLOTS + kg * (IN_ROWS * ROW_SLOTS);
-    const u32x4* wt = lds_w + ((size_t)wstep * 2 + kg) * MT + ln;
+    const u32x4* wt = lds_w + kg * (WTAPS * MT) + ln + wstep * (2 * WTAPS * MT);
     const int col = tpart < 2 ? 32 * tpart + ln + p.lead : ln - p.extra_w;
     auto product = [&](int tap, int row, int kw) __attribute__((always_inline)) {
-      const u32x4 a = wt[(size_t)tap * p.wc16 * 2 * MT], v = in[row * ROW_SLOTS + in_slot(max(col + kw, 0))];
+      const u32x4 a = wt[tap * MT], v = in[row * ROW_SLOTS + in_slot(max(col + kw, 0))];
       const u32x4 b = col + kw < 0 ? u32x4{0u, 0u, 0u, 0u} : v;
       top = F16 ? __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), top, 0, 0, 0)
                 : __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), top, 0, 0, 0);

@@ -298,8 +298,8 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
   // (pair 0: the rows shared with the stage above, pair 1: the two new rows).
   // Position of a stage: row pair (fastest), column tile, output depth, batch entry, and the first bytes of its g rows and its new x
   // rows. Decoded once, then stepped: down a strip the two addresses move by a constant, and only a new strip works
-  // them out. (From scratch in every stage they were most of its 116 scalar instructions, whose issue no matrix instruction of the
-  // SIMD's other wavefront hides: SCALAR_FIGURES.)
+  // them out. (From scratch in every stage they were most of its 120 to 170 scalar instructions: 2 x 40 -> 72 of 217 x 301 37.2 -> 34.6 us,
+  // 2 x 48 -> 19 of 121 x 126 x 78 538 -> 509, 2 x 32 -> 32 of 128^3 284 -> 268; 64 x 64 blocks without edges do not wait for them, 617 -> 615.)
   struct Cursor {
     int hp, ct, od, n;
     const char *g, *x;
@@ -858,7 +858,7 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
 // block's partial (a tap, a pair, four registers and 64 / SUB lanes of the kernel above), a lane four of them; its 8 wavefronts
 // take 8 SUB partials at a time in chains of their own and the sums are added in a fixed order (deterministic). What bounds it is
 // the latency of the chains, 16-byte loads, eight in flight a lane: a block of 32 x 32 is 36 runs of 256 values, which left most of
-// the chip idle (reduce_subs; RED_FIGURES).
+// the chip idle (reduce_subs): 6 x 26 -> 27 of 197 x 140 12.4 us, cut in four 6.6.
 // The workgroups behind those of the last block add up bias partials, 16 channels each, four partials a wavefront at a time.
 struct ReduceParams {
   const float* part;
