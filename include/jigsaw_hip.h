@@ -592,6 +592,26 @@ int jg_conv_wgrad_bias(void* gw, void* gb, const void* x, const void* g,
                        const jg_conv_desc* desc, int dtype, void* workspace,
                        size_t workspace_bytes, void* stream);
 
+/* jg_conv_wgrad_bias whose sums over the workgroups' partials are left for later: `later` (set by the call) says what is left, kind 0
+ * nothing. jg_conv_reduce or jg_halo_fold_border_reduce_3d does it, on a stream ordered behind the call and with the bits of
+ * jg_conv_wgrad_bias; until then workspace, gw and gb stay where they are. */
+typedef struct jg_conv_reduction {
+  int32_t kind, dtype; /* the library's own, as all of it */
+  const float* part;
+  const float* bias_part;
+  void* gw;
+  void* gb;
+  int32_t runs, sub, slots, npairs, pairs, rows, cols, ci_step, ci_blocks, KD, cin, cout, bias_cout, bias_parts;
+} jg_conv_reduction;
+int jg_conv_wgrad_bias_later(jg_conv_reduction* later, void* gw, void* gb, const void* x, const void* g,
+                             const jg_conv_desc* desc, int dtype, void* workspace, size_t workspace_bytes, void* stream);
+int jg_conv_reduce(const jg_conv_reduction* later, void* stream);
+/* jg_halo_fold_border_3d, and what `later` holds in the same launch where jg_halo_fold_border_takes_sums says so (1; 0 where it takes a
+ * launch of its own and is better done while the partials are in the caches). */
+int jg_halo_fold_border_takes_sums(const jg_halo_geom* geom, int dtype);
+int jg_halo_fold_border_reduce_3d(void* gx, const void* const strips[27], const jg_halo_geom* geom, int dtype,
+                                  const jg_conv_reduction* later, void* stream);
+
 /* gb (C,) = sum of g (N, C, spatial...) over batch and spatial axes —
  * _sum_grad_bias, jigsaw/modules/convolution/_conv/config.py:117-120.
  * `spatial` = product of the spatial extents. */

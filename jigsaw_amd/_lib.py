@@ -273,6 +273,13 @@ SIGNATURES: dict[str, tuple] = {
         c_int,
         [c_void_p, c_void_p, c_void_p, c_void_p, POINTER(ConvDesc), c_int, c_void_p, c_size_t, c_void_p],
     ),
+    "jg_conv_wgrad_bias_later": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, POINTER(ConvDesc), c_int, c_void_p, c_size_t, c_void_p],
+    ),
+    "jg_conv_reduce": (c_int, [c_void_p, c_void_p]),
+    "jg_halo_fold_border_takes_sums": (c_int, [POINTER(HaloGeom), c_int]),
+    "jg_halo_fold_border_reduce_3d": (c_int, [c_void_p, POINTER(c_void_p), POINTER(HaloGeom), c_int, c_void_p, c_void_p]),
     "jg_bias_grad_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64]),
     "jg_bias_grad": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p, c_size_t, c_void_p]),
     "jg_attn_fwd": (

@@ -1097,13 +1097,13 @@ def conv_halo_nway_backward(
         stream = _lib.stream_handle(g.device) if step is not None else 0
         parts = step.backward(g, x_aug, weight, need_x, need_w, need_w and need_b, stream) if step is not None else None
         if parts is not None:
-            part, g_w, g_b, send, folded = parts
+            part, g_w, g_b, send, folded, left = parts
             if need_b and g_b is None:
                 g_b = config.grad_bias(g.contiguous())
             if not need_x:
                 return done(None)
             recv = config.halo_exchange.backward(send) if step.sends else {}
-            g_x = step.finish(part, folded, recv, stream)
+            g_x = step.finish(part, folded, recv, stream, left)
             if g_x is None:
                 geom = HaloGeometry.for_conv(local_in_spatial, weight.shape[-n:], stride, padding, dilation, ranks, sizes)
                 g_x = halo_fold_border_(part, recv, geom) if folded else halo_fold(part, recv, geom)

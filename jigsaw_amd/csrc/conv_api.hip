@@ -2,6 +2,7 @@
 // route to the implicit-GEMM MFMA kernels when they cover the problem, to the
 // direct kernels otherwise.
 #include "conv_common.h"
+#include "conv_reduce.h"
 
 namespace jg {
 
@@ -199,17 +200,41 @@ extern "C" int jg_conv_wgrad_framed(void* gw, void* gb, const void* x_frame, con
                         x_tile, tlo, tn);
 }
 
-extern "C" int jg_conv_wgrad_bias(void* gw, void* gb, const void* x, const void* go,
-                                  const jg_conv_desc* desc, int dtype, void* workspace,
-                                  size_t workspace_bytes, void* stream) {
+static int wgrad_bias(jg_conv_reduction* later, void* gw, void* gb, const void* x, const void* go, const jg_conv_desc* desc, int dtype,
+                      void* workspace, size_t workspace_bytes, void* stream) {
   jg::ConvGeom g;
   int rc = jg::resolve_conv(desc, "jg_conv_wgrad_bias", &g);
   if (rc) return rc;
   JG_REQUIRE(gw && gb && x && go, "jg_conv_wgrad_bias: NULL pointer");
   JG_REQUIRE(known(dtype), "jg_conv_wgrad_bias: unknown dtype %d", dtype);
-  if (jg::f32_conv_supported(g, dtype)) return jg::f32_wgrad(gw, gb, x, go, g, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+  if (jg::f32_conv_supported(g, dtype)) return jg::f32_wgrad(gw, gb, x, go, g, workspace, workspace_bytes, static_cast<hipStream_t>(stream), later);
   if (!jg::mfma_wgrad_supported(g, dtype))
     JG_FAIL(JG_ERR_UNSUPPORTED, "jg_conv_wgrad_bias: geometry only has the separate kernels");
   return jg::mfma_wgrad(gw, gb, x, go, g, workspace, workspace_bytes, static_cast<hipStream_t>(stream), nullptr, nullptr, nullptr,
-                        dtype);
+                        dtype, later);
+}
+
+extern "C" int jg_conv_wgrad_bias(void* gw, void* gb, const void* x, const void* go,
+                                  const jg_conv_desc* desc, int dtype, void* workspace,
+                                  size_t workspace_bytes, void* stream) {
+  return wgrad_bias(nullptr, gw, gb, x, go, desc, dtype, workspace, workspace_bytes, stream);
+}
+
+extern "C" int jg_conv_wgrad_bias_later(jg_conv_reduction* later, void* gw, void* gb, const void* x, const void* go, const jg_conv_desc* desc,
+                                        int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  JG_REQUIRE(later != nullptr, "jg_conv_wgrad_bias_later: NULL pointer");
+  memset(later, 0, sizeof(*later));
+  return wgrad_bias(later, gw, gb, x, go, desc, dtype, workspace, workspace_bytes, stream);
+}
+
+int jg::conv_reduce(const jg_conv_reduction& later, hipStream_t s) {
+  if (later.kind == CONV_REDUCE_TILES) return tiles_reduce(later, s);
+  if (later.kind == CONV_REDUCE_F32) return f32_reduce(later, s);
+  JG_REQUIRE(later.kind == CONV_REDUCE_NONE, "jg_conv_reduce: unknown kind %d", later.kind);
+  return JG_OK;
+}
+
+extern "C" int jg_conv_reduce(const jg_conv_reduction* later, void* stream) {
+  JG_REQUIRE(later != nullptr, "jg_conv_reduce: NULL pointer");
+  return jg::conv_reduce(*later, static_cast<hipStream_t>(stream));
 }

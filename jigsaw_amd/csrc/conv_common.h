@@ -53,14 +53,17 @@ int mfma_dgrad_fold(void* gx, void* const strips[27], const int lo[3], const int
 // xt / tlo / tn: framed input as for mfma_fwd_framed, or NULL
 int mfma_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom& g, void* ws,
                size_t ws_bytes, hipStream_t s, const void* xt = nullptr, const int* tlo = nullptr,
-               const int* tn = nullptr, int dtype = JG_BF16);
+               const int* tn = nullptr, int dtype = JG_BF16, jg_conv_reduction* later = nullptr);
+int tiles_reduce(const jg_conv_reduction& later, hipStream_t s);
+int f32_reduce(const jg_conv_reduction& later, hipStream_t s);
 // fp32 3 x 3 layers on the fp32 matrix instruction (conv_f32.hip). Neither the forward nor the input gradient takes a workspace;
 // lo / n: as for mfma_dgrad_fold, or NULL.
 bool f32_conv_supported(const ConvGeom& g, int dtype);
 int f32_fwd(void* y, const void* x, const void* w, const void* bias, const ConvGeom& g, hipStream_t s);
 int f32_dgrad(void* gx, void* const* strips, const int* lo, const int* n, const void* w, const void* go, const ConvGeom& g, hipStream_t s);
 size_t f32_wgrad_workspace(const ConvGeom& g);
-int f32_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom& g, void* ws, size_t ws_bytes, hipStream_t s);
+int f32_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom& g, void* ws, size_t ws_bytes, hipStream_t s,
+              jg_conv_reduction* later = nullptr);
 // dst (batch, parts, per_batch) bf16 = the bf16 parts of src (batch, per_batch), whose sum is src:
 // three for fp32, two for fp16. The operand layout of the split mode of the MFMA kernels.
 int split_parts_bf16(uint16_t* dst, const void* src, int src_dtype, size_t batch, size_t per_batch, hipStream_t s);

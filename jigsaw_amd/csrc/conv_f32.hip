@@ -20,6 +20,7 @@
 // with many channels the instruction's rate, 74 of 157 TFLOP/s at 20 -> 20 channels, 8 x 500^2. f32_conv_supported has the line
 // between the two. Against float64 no result is further off than the three parts' (relative, 16 channels: y 1.9e-7 : 2.5e-7).
 #include "conv_common.h"
+#include "conv_reduce.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -346,32 +347,10 @@ __global__ __launch_bounds__(THREADS) void wgrad_f32_kernel(WgradParams p) {
       for (int i = 0; i < 4; ++i) out[(mt * 16 + i) * COLS + nb * 16] = (float)total[mt][nb][i];
 }
 
-// gw and gb from the slots of every block: 64 neighbouring values a workgroup, sixteen chains of slots, added in order
-constexpr int CHAINS = 16;
-__global__ __launch_bounds__(64 * CHAINS) void wgrad_f32_reduce_kernel(float* gw, float* gb, const float* __restrict__ part, int slots, int rows,
-                                                                       int cols, int CI, int M, int C, int ci_blocks) {
-  __shared__ double red[CHAINS][64];
-  const int lane = threadIdx.x & 63, chain = threadIdx.x >> 6, per_block = rows * cols / 64;
-  const int block = blockIdx.x / per_block, at = (blockIdx.x - block * per_block) * 64 + lane;
-  const size_t stride = (size_t)rows * cols;
-  const float* src = part + (size_t)block * slots * stride + at;
-  double s[4] = {};
-  int k = chain;
-  for (; k + 3 * CHAINS < slots; k += 4 * CHAINS)
-#pragma unroll
-    for (int u = 0; u < 4; ++u) s[u] += src[(size_t)(k + u * CHAINS) * stride];
-  for (; k < slots; k += CHAINS) s[0] += src[(size_t)k * stride];
-  red[chain][lane] = (s[0] + s[1]) + (s[2] + s[3]);
-  __syncthreads();
-  if (chain != 0) return;
-  double total = 0.0;
-#pragma unroll
-  for (int u = 0; u < CHAINS; ++u) total += red[u][lane];
-  const float sum = (float)total;
-  const int co = block / ci_blocks * rows + at / cols, j = at % cols, ci = block % ci_blocks * CI + j / 9;
-  if (co >= M) return;
-  if (j < CI * 9 && ci < C) gw[((size_t)co * C + ci) * 9 + j % 9] = sum;
-  if (j == CI * 9 && block % ci_blocks == 0 && gb != nullptr) gb[co] = sum;
+constexpr int REDUCE_THREADS = 64 * jg::CONV_RED_CHAINS;
+__global__ __launch_bounds__(REDUCE_THREADS) void wgrad_f32_reduce_kernel(jg_conv_reduction p) {
+  __shared__ jg::ConvReduceShared shared;
+  jg::reduce_conv_f32<jg::CONV_RED_CHAINS>(p, blockIdx.x, shared);
 }
 
 // The weight gradient's blocks: input channels of a block, 16 MT output channels, workgroups of a block
@@ -471,7 +450,8 @@ int f32_dgrad(void* gx, void* const* strips, const int* lo, const int* n, const 
 
 size_t f32_wgrad_workspace(const ConvGeom& g) { return plan_of(g).bytes(); }
 
-int f32_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom& g, void* ws, size_t ws_bytes, hipStream_t s) {
+int f32_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom& g, void* ws, size_t ws_bytes, hipStream_t s,
+              jg_conv_reduction* later) {
   const char* who = "jg_conv_wgrad(fp32)";
   const Plan q = plan_of(g);
   if (ws == nullptr || ws_bytes < q.bytes()) JG_FAIL(JG_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, ws_bytes, q.bytes());
@@ -490,10 +470,21 @@ int f32_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom&
   else kern = q.MT == 2 ? &wgrad_f32_kernel<2, 1, 4> : &wgrad_f32_kernel<1, 1, 4>;
   kern<<<grid, THREADS, 0, s>>>(p);
   JG_CHECK_LAUNCH(who);
-  const int rows = q.MT * 16;
-  wgrad_f32_reduce_kernel<<<(unsigned)(blocks * (rows * q.cols / 64)), 64 * CHAINS, 0, s>>>(
-      static_cast<float*>(gw), static_cast<float*>(gb), p.part, q.wgs * q.rs, rows, q.cols, q.CI, g.cout, g.cin, q.ci_blocks);
-  JG_CHECK_LAUNCH(who);
+  jg_conv_reduction r = {};
+  r.kind = CONV_REDUCE_F32;
+  r.dtype = JG_F32;
+  r.part = p.part; r.gw = gw; r.gb = gb;
+  r.slots = q.wgs * q.rs; r.rows = q.MT * 16; r.cols = q.cols; r.ci_step = q.CI; r.ci_blocks = q.ci_blocks;
+  r.cin = g.cin; r.cout = g.cout;
+  r.runs = blocks * (r.rows * q.cols / CONV_F32_VALUES);
+  if (later == nullptr) return f32_reduce(r, s);
+  *later = r;
+  return JG_OK;
+}
+
+int f32_reduce(const jg_conv_reduction& r, hipStream_t s) {
+  wgrad_f32_reduce_kernel<<<conv_reduce_blocks(r), REDUCE_THREADS, 0, s>>>(r);
+  JG_CHECK_LAUNCH("jg_conv_wgrad(fp32 reduce)");
   return JG_OK;
 }
 

@@ -40,9 +40,9 @@
 //               (deterministic) and writes gw in the weight layout and gb, in their own dtype.
 #include <algorithm>
 #include <cmath>
-#include <type_traits>
 
 #include "conv_common.h"
+#include "conv_reduce.h"
 
 namespace {
 
@@ -853,106 +853,10 @@ __global__ __launch_bounds__(wgrad_threads(CGB, CXB), wgrad_waves_per_simd(CGB, 
   }
 }
 
-// gw = sum over the partials of a block of channels (its workgroups, and in split mode its part pairs, which
-// lie behind each other), and gb the same over the bias partials. A workgroup owns a run of 256 / SUB values of a
-// block's partial (a tap, a pair, four registers and 64 / SUB lanes of the kernel above), a lane four of them; its 8 wavefronts
-// take 8 SUB partials at a time in chains of their own and the sums are added in a fixed order (deterministic). What bounds it is
-// the latency of the chains, 16-byte loads, eight in flight a lane: a block of 32 x 32 is 36 runs of 256 values, which left most of
-// the chip idle (reduce_subs): 6 x 26 -> 27 of 197 x 140 12.4 us, cut in four 6.6.
-// The workgroups behind those of the last block add up bias partials, 16 channels each, four partials a wavefront at a time.
-struct ReduceParams {
-  const float* part;
-  const float* bias_part;
-  void* gw;
-  void* gb;
-  int wgs, npairs;            // workgroups of a block, part pairs
-  int pairs, GC, CXB, cin_b;  // 32 x 32 pairs of a block; its g channels, x blocks and x channels per depth tap
-  int KD, cin, cout, ci_blocks;
-  int gw_blocks;              // workgroups that reduce gw
-  int bias_cout, bias_parts;  // output channels, and parts of g whose bias sums belong together
-};
-constexpr int RED_WAVES = 8, BIAS_CHANNELS = 16;
-template <int OUT>  // dtype of gw and gb: 0 bf16, 1 fp32, 2 fp16
-__device__ __forceinline__ void store_gradient(void* out, size_t at, float v) {
-  if (OUT == 1) static_cast<float*>(out)[at] = v;
-  else if (OUT == 2) static_cast<_Float16*>(out)[at] = (_Float16)v;
-  else static_cast<uint16_t*>(out)[at] = jg::f32_to_bf16(v);
-}
-template <int OUT, int SUB>
-__global__ __launch_bounds__(64 * RED_WAVES) void wgrad_reduce_kernel(ReduceParams p) {
-  constexpr int LANES = 64 / SUB, CHAINS = RED_WAVES * SUB;  // lanes of a run, chains of a workgroup
-  __shared__ f32x4 red[RED_WAVES][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if ((int)blockIdx.x >= p.gw_blocks) {
-    // bias: a channel's block at x block 0 and x part 0 holds its sums
-    const int c = ((int)blockIdx.x - p.gw_blocks) * BIAS_CHANNELS + lane % BIAS_CHANNELS, first = w * (64 / BIAS_CHANNELS) + lane / BIAS_CHANNELS;
-    constexpr int STEP = RED_WAVES * (64 / BIAS_CHANNELS);
-    float s = 0.0f;
-    if (c < p.bias_cout) {
-      for (int gp = p.bias_parts - 1; gp >= 0; --gp) {
-        // plain: one pair per block. Part pairs: the pair (gp, 0) is pair kBias of the block
-        const int pair_k = p.npairs == 6 ? (gp == 2 ? 2 : (gp == 1 ? 4 : 5)) : 0;
-        const int row = p.npairs == 1 ? gp * p.bias_cout + c : c;  // all parts in one block: parts are channels of it
-        const size_t slot0 = ((size_t)(row / p.GC) * p.ci_blocks * p.npairs + pair_k) * p.wgs;
-        const float* src = p.bias_part + slot0 * p.GC + row % p.GC;
-        float c8[8] = {};
-        for (int k = first; k < p.wgs; k += 8 * STEP) {
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            const int at = k + u * STEP;
-            c8[u] += at < p.wgs ? src[(size_t)at * p.GC] : 0.0f;
-          }
-        }
-        s += ((c8[0] + c8[1]) + (c8[2] + c8[3])) + ((c8[4] + c8[5]) + (c8[6] + c8[7]));
-      }
-    }
-#pragma unroll
-    for (int o = BIAS_CHANNELS; o < 64; o <<= 1) s += __shfl_xor(s, o, 64);
-    red[w][lane].x = s;
-    __syncthreads();
-    if (w != 0 || lane >= BIAS_CHANNELS || c >= p.bias_cout) return;
-    s = 0.0f;
-#pragma unroll
-    for (int k = 0; k < RED_WAVES; ++k) s += red[k][lane].x;
-    store_gradient<OUT>(p.gb, c, s);
-    return;
-  }
-  const int runs = 9 * p.pairs * 4;  // runs of 256 values in a block's partial
-  const int own = blockIdx.x / SUB, blk = own / runs, run = own - blk * runs;
-  const int at = (int)(blockIdx.x % SUB) * LANES + lane % LANES;  // the lane of the kernel above whose values these are
-  const int slots = p.wgs * p.npairs;
-  const size_t stride = (size_t)runs * 256;
-  const float* src = p.part + (size_t)blk * slots * stride + (size_t)run * 256 + at * 4;
-  f32x4 c[8] = {};
-  int k = w * SUB + lane / LANES;
-  for (; k + 7 * CHAINS < slots; k += 8 * CHAINS) {
-#pragma unroll
-    for (int u = 0; u < 8; ++u) c[u] += *reinterpret_cast<const f32x4*>(src + (size_t)(k + u * CHAINS) * stride);
-  }
-#pragma unroll
-  for (int u = 0; u < 7; ++u)
-    if (k + u * CHAINS < slots) c[u] += *reinterpret_cast<const f32x4*>(src + (size_t)(k + u * CHAINS) * stride);
-  f32x4 sum = ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
-#pragma unroll
-  for (int o = LANES; o < 64; o <<= 1)
-#pragma unroll
-    for (int u = 0; u < 4; ++u) sum[u] += __shfl_xor(sum[u], o, 64);
-  red[w][lane] = sum;
-  __syncthreads();
-  if (w != 0 || lane >= LANES) return;
-  sum = red[0][lane];
-#pragma unroll
-  for (int u = 1; u < RED_WAVES; ++u) sum += red[u][lane];
-  const int j = run & 3, pair = (run >> 2) % p.pairs, tap = (run >> 2) / p.pairs;
-  const int cb = pair / p.CXB, ib = pair % p.CXB;
-  const int cx = ib * 32 + (at & 31), kd = cx / p.cin_b;
-  const int ci = (blk % p.ci_blocks) * p.cin_b + cx % p.cin_b;
-  if (ci >= p.cin) return;
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int co = (blk / p.ci_blocks) * p.GC + cb * 32 + 8 * j + 4 * (at >> 5) + u;
-    if (co < p.cout) store_gradient<OUT>(p.gw, (((size_t)co * p.cin + ci) * p.KD + kd) * 9 + tap, sum[u]);
-  }
+template <int DT>
+__global__ __launch_bounds__(64 * jg::CONV_RED_WAVES) void wgrad_reduce_kernel(jg_conv_reduction p) {
+  __shared__ jg::ConvReduceShared shared;
+  jg::reduce_conv_tiles<DT>(p, blockIdx.x, shared);
 }
 
 // gw[co][ci][t] (fp32) = sum over the part pairs (i, j), i + j <= parts - 1, smallest first, of
@@ -1041,10 +945,10 @@ Plan plan_of(const ConvGeom& g, int parts) {
   return p;
 }
 
-// Pieces that a run of 256 values is cut into: up to two workgroups a compute unit.
-int reduce_subs(long long runs) {
+// Pieces (their logarithm) that a run of 256 values is cut into: up to two workgroups a compute unit.
+int reduce_sub(long long runs) {
   const long long most = 2ll * jg::cu_count();
-  return 4 * runs <= most ? 4 : 2 * runs <= most ? 2 : 1;
+  return 4 * runs <= most ? 2 : 2 * runs <= most ? 1 : 0;
 }
 
 template <int CGB, int CXB>
@@ -1130,8 +1034,17 @@ bool mfma_wgrad_frame_ok(const ConvGeom& g, const int tlo[3], const int tn[3]) {
   return true;
 }
 
+int tiles_reduce(const jg_conv_reduction& r, hipStream_t s) {
+  const unsigned grid = conv_reduce_blocks(r);
+  if (r.dtype == JG_F32) wgrad_reduce_kernel<JG_F32><<<grid, 64 * CONV_RED_WAVES, 0, s>>>(r);
+  else if (r.dtype == JG_F16) wgrad_reduce_kernel<JG_F16><<<grid, 64 * CONV_RED_WAVES, 0, s>>>(r);
+  else wgrad_reduce_kernel<JG_BF16><<<grid, 64 * CONV_RED_WAVES, 0, s>>>(r);
+  JG_CHECK_LAUNCH("jg_conv_wgrad(reduce)");
+  return JG_OK;
+}
+
 int mfma_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom& g, void* ws,
-               size_t ws_bytes, hipStream_t s, const void* xt, const int* tlo, const int* tn, int dtype) {
+               size_t ws_bytes, hipStream_t s, const void* xt, const int* tlo, const int* tn, int dtype, jg_conv_reduction* later) {
   const char* who = "jg_conv_wgrad(mfma)";
   if (!covered(g)) JG_FAIL(JG_ERR_UNSUPPORTED, "%s: geometry not covered", who);
   if (ws == nullptr || ws_bytes < mfma_wgrad_workspace(g, dtype))
@@ -1209,29 +1122,24 @@ int mfma_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom
   if (rc) return rc;
   JG_CHECK_LAUNCH(who);
 
-  ReduceParams r;
+  jg_conv_reduction r = {};
+  r.kind = jg::CONV_REDUCE_TILES;
+  r.dtype = dtype;
   r.part = p.part; r.bias_part = p.bias_part;
   r.gw = plan.parts_in_block > 1 ? one_block_tmp : gw;
   r.gb = gb;
-  r.wgs = plan.wgs; r.npairs = plan.npairs;
-  r.pairs = plan.cgb * plan.cxb; r.GC = (int)plan.GC(); r.CXB = plan.cxb; r.cin_b = (int)plan.XC() / plan.KD;
+  r.slots = plan.wgs; r.npairs = plan.npairs;
+  r.pairs = plan.cgb * plan.cxb; r.rows = (int)plan.GC(); r.cols = plan.cxb; r.ci_step = (int)plan.XC() / plan.KD;
   r.KD = plan.KD; r.cin = p.cin; r.cout = p.cout; r.ci_blocks = plan.ci_blocks;
   r.bias_cout = g.cout; r.bias_parts = parts;
-  r.gw_blocks = plan.co_blocks * plan.ci_blocks * 9 * r.pairs * 4;
-  const unsigned bgrid = gb != nullptr ? (unsigned)(g.cout + BIAS_CHANNELS - 1) / BIAS_CHANNELS : 0u;
-  auto reduce = [&](auto sub) {
-    constexpr int SUB = decltype(sub)::value;
-    r.gw_blocks *= SUB;
-    const unsigned rgrid = (unsigned)r.gw_blocks + bgrid;
-    if (dtype == JG_F32) wgrad_reduce_kernel<1, SUB><<<rgrid, 64 * RED_WAVES, 0, s>>>(r);
-    else if (f16) wgrad_reduce_kernel<2, SUB><<<rgrid, 64 * RED_WAVES, 0, s>>>(r);
-    else wgrad_reduce_kernel<0, SUB><<<rgrid, 64 * RED_WAVES, 0, s>>>(r);
-  };
-  const int subs = reduce_subs(r.gw_blocks);
-  if (subs == 4) reduce(std::integral_constant<int, 4>{});
-  else if (subs == 2) reduce(std::integral_constant<int, 2>{});
-  else reduce(std::integral_constant<int, 1>{});
-  JG_CHECK_LAUNCH(who);
+  r.runs = plan.co_blocks * plan.ci_blocks * 9 * r.pairs * 4;
+  r.sub = reduce_sub(r.runs);
+  if (later != nullptr && plan.parts_in_block == 1) {
+    *later = r;
+    return JG_OK;
+  }
+  rc = tiles_reduce(r, s);
+  if (rc) return rc;
   if (plan.parts_in_block > 1) {
     // few channels: all part products came from one block (the parts are channels of it); the ones that count
     // are added up

@@ -9,7 +9,7 @@
 //   jigsaw/modules/convolution/_conv/halo.py:66-156   (halo_gather)
 //   jigsaw/modules/convolution/_conv/halo.py:159-251  (halo_scatter_add)
 //   jigsaw/modules/convolution/_conv/distributed.py:264-275, 378-389 (axis order)
-#include "jg_common.h"
+#include "conv_reduce.h"
 
 namespace {
 
@@ -1043,17 +1043,17 @@ __device__ __forceinline__ void fold_border_span(typename Arith<DT>::T* drow, co
 }
 
 template <int DT>
-__device__ __forceinline__ void fold_border_rows(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp) {
+__device__ __forceinline__ void fold_border_rows(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp, unsigned block, unsigned thread) {
   typedef typename Arith<DT>::T T;
   constexpr int V = Bits<T>::V;
   // a row is owned by bp.lpr lanes (a power of two up to 64: a whole wavefront for long rows)
-  const uint32_t item = ((blockIdx.x - bp.edge_blocks) * 256u + threadIdx.x) / (uint32_t)bp.lpr;
+  const uint32_t item = ((block - bp.edge_blocks) * 256u + thread) / (uint32_t)bp.lpr;
   if (item >= bp.row_items) return;
   int d, h;
   const long long p = (long long)border_row(item, g, bp, d, h);
   const int W = g.n[2], up0 = W - g.lo[2];
   T* drow = gx + ((p * g.n[0] + d) * g.n[1] + h) * (long long)W;
-  for (int c0 = (threadIdx.x & (bp.lpr - 1)) * V; c0 < up0; c0 += bp.lpr * V) {
+  for (int c0 = (thread & (bp.lpr - 1)) * V; c0 < up0; c0 += bp.lpr * V) {
     const int b = max(c0, bp.head), e = min(c0 + V, up0);
     if (b < e) fold_border_span<DT>(drow, g, p, d, h, c0, b, e);
   }
@@ -1061,9 +1061,9 @@ __device__ __forceinline__ void fold_border_rows(typename Arith<DT>::T* __restri
 
 // The edge columns of such a row, one lane per cell
 template <int DT>
-__device__ __forceinline__ void fold_border_edges(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp) {
+__device__ __forceinline__ void fold_border_edges(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp, unsigned block, unsigned thread) {
   typedef typename Arith<DT>::T T;
-  const uint32_t at = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t at = block * 256u + thread;
   if (at >= bp.edge_items) return;
   const uint32_t item = mdiv(at, bp.div_edge);
   const int q = (int)(at - item * (uint32_t)bp.n_edge);
@@ -1102,9 +1102,9 @@ __device__ __forceinline__ void fold_border_edges(typename Arith<DT>::T* __restr
 }
 
 template <int DT>
-__device__ __forceinline__ void fold_border_cols(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp) {
+__device__ __forceinline__ void fold_border_cols(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp, unsigned block, unsigned thread) {
   typedef typename Arith<DT>::T T;
-  const uint32_t item = (blockIdx.x - bp.edge_blocks - bp.row_blocks) * 256u + threadIdx.x;  // (row, edge cell), cell fastest
+  const uint32_t item = (block - bp.edge_blocks - bp.row_blocks) * 256u + thread;  // (row, edge cell), cell fastest
   if (item >= bp.col_items) return;
   const int D = g.n[0], H = g.n[1], W = g.n[2];
   const uint32_t row = mdiv(item, bp.div_edge);
@@ -1130,10 +1130,31 @@ __device__ __forceinline__ void fold_border_cols(typename Arith<DT>::T* __restri
 
 // tab comes first among the parameters: its entries are read from the kernel-argument segment
 template <int DT>
+__device__ __forceinline__ void fold_border_block(typename Arith<DT>::T* __restrict__ gx, const Geom& g, const BorderPlan& bp, unsigned block, unsigned thread) {
+  if (block < bp.edge_blocks) fold_border_edges<DT>(gx, g, bp, block, thread);
+  else if (block < bp.edge_blocks + bp.row_blocks) fold_border_rows<DT>(gx, g, bp, block, thread);
+  else fold_border_cols<DT>(gx, g, bp, block, thread);
+}
+template <int DT>
 __global__ __launch_bounds__(256) void fold_border_kernel(Table tab, typename Arith<DT>::T* __restrict__ gx, Geom g, BorderPlan bp) {
-  if (blockIdx.x < bp.edge_blocks) fold_border_edges<DT>(gx, g, bp);
-  else if (blockIdx.x < bp.edge_blocks + bp.row_blocks) fold_border_rows<DT>(gx, g, bp);
-  else fold_border_cols<DT>(gx, g, bp);
+  fold_border_block<DT>(gx, g, bp, blockIdx.x, threadIdx.x);
+}
+
+// The border cells, and in front of them the sums that a convolution's weight gradient left (conv_reduce.h). Each alone is a launch of 4 to
+// 13 us that fills a fraction of the chip and waits for its own latency. Together, for the two (the sums cut as there): 2 x 40 -> 72 of
+// 217 x 301 10.6 -> 6.6 us, 64 -> 128 of 4 x 256^2 at stride 2 12.8 -> 9.8, 8 x 4 -> 8 of 242 x 233 17.5 -> 7.2, fp32 4 x 3 -> 16 of
+// 256^2 11.6 -> 4.6. (Workgroups of four wavefronts that walk the chains of eight: 13.5 for the third of them, out of registers.)
+template <int DT>
+__global__ __launch_bounds__(512) void fold_border_reduce_kernel(Table tab, typename Arith<DT>::T* __restrict__ gx, Geom g, BorderPlan bp,
+                                                                 jg_conv_reduction later, unsigned reduce_blocks) {
+  __shared__ jg::ConvReduceShared shared;
+  if (blockIdx.x < reduce_blocks) {
+    if (DT == JG_F32 && later.kind == jg::CONV_REDUCE_F32) jg::reduce_conv_f32<8>(later, blockIdx.x, shared);
+    else jg::reduce_conv_tiles<DT>(later, blockIdx.x, shared);
+    return;
+  }
+  // two blocks of the border (the cells end with the last one, or before the second half of it)
+  fold_border_block<DT>(gx, g, bp, 2 * (blockIdx.x - reduce_blocks) + (threadIdx.x >> 8), threadIdx.x & 255);
 }
 
 Magic make_magic(uint32_t d) {
@@ -1489,14 +1510,22 @@ bool border_plan(const Geom& g, BorderPlan* bp, unsigned long long* row_items, u
   *col_items = nrows * (unsigned long long)bp->n_edge;
   return *row_items < (1ull << 31) && *col_items < (1ull << 31) && nrows < (1ull << 31);
 }
+int border_lanes(const Geom& g, int elem_size) {  // of a row
+  const int V = 16 / elem_size, vecs = (g.n[2] - g.lo[2] + V - 1) / V;
+  int lanes = 1;
+  while (lanes < 64 && lanes < vecs) lanes *= 2;
+  return lanes;
+}
+unsigned long long border_blocks(const Geom& g, int dtype, const BorderPlan& bp, unsigned long long row_items, unsigned long long col_items) {
+  const unsigned long long lanes = border_lanes(g, (int)jg::dtype_size(dtype));
+  return (row_items * bp.n_edge + 255) / 256 + (row_items * lanes + 255) / 256 + (col_items + 255) / 256;
+}
 // The rows a D or H neighbour reaches, summed in full in place; false if there are too many.
 template <int DT>
 bool launch_border(const Table& tab, void* gx, const Geom& g, BorderPlan bp, unsigned long long row_items,
-                   unsigned long long col_items, hipStream_t s) {
+                   unsigned long long col_items, hipStream_t s, const jg_conv_reduction* later = nullptr) {
   typedef typename Arith<DT>::T T;
-  const int V = 16 / (int)sizeof(T), vecs = (g.n[2] - g.lo[2] + V - 1) / V;
-  bp.lpr = 1;
-  while (bp.lpr < 64 && bp.lpr < vecs) bp.lpr *= 2;
+  bp.lpr = border_lanes(g, (int)sizeof(T));
   const unsigned long long threads = row_items * (unsigned long long)bp.lpr, edge_items = row_items * (unsigned long long)bp.n_edge;
   if (threads >= (1ull << 32) || edge_items >= (1ull << 31) || col_items >= (1ull << 32)) return false;
   bp.edge_items = (uint32_t)edge_items;
@@ -1506,6 +1535,11 @@ bool launch_border(const Table& tab, void* gx, const Geom& g, BorderPlan bp, uns
   bp.row_blocks = (uint32_t)((threads + 255) / 256);
   const unsigned long long blocks = bp.edge_blocks + bp.row_blocks + (col_items + 255) / 256;
   if (blocks == 0) return true;
+  if (later != nullptr && later->kind != jg::CONV_REDUCE_NONE) {
+    const unsigned sums = jg::conv_reduce_blocks(*later);
+    fold_border_reduce_kernel<DT><<<(unsigned)(blocks + 1) / 2 + sums, 512, 0, s>>>(tab, static_cast<T*>(gx), g, bp, *later, sums);
+    return true;
+  }
   fold_border_kernel<DT><<<(unsigned)blocks, 256, 0, s>>>(tab, static_cast<T*>(gx), g, bp);
   return true;
 }
@@ -1587,8 +1621,22 @@ extern "C" int jg_halo_fold_3d(void* gx, const void* gx_aug, const void* const s
   return JG_OK;
 }
 
-extern "C" int jg_halo_fold_border_3d(void* gx, const void* const strips[27],
-                                      const jg_halo_geom* geom, int dtype, void* stream) {
+// What is left of a weight gradient goes into the launch of the border while that one's blocks fit the chip at once and both are
+// latency. The many cells of a volume's faces keep their own kernel, with fewer registers and more wavefronts in flight, and large
+// partials are better read right behind the kernel that wrote them: 8 x 64 -> 64 of 1024^2 10 us there, 18 behind the input gradient.
+static bool takes_sums(const Geom& g, int dtype) {
+  BorderPlan bp;
+  unsigned long long row_items = 0, col_items = 0;
+  if (g.planes <= 0 || g.n[0] <= 0 || g.n[1] <= 0 || g.n[2] <= 0 || !border_plan(g, &bp, &row_items, &col_items)) return false;
+  return row_items + col_items != 0 && border_blocks(g, dtype, bp, row_items, col_items) <= 8ull * jg::cu_count();
+}
+
+extern "C" int jg_halo_fold_border_takes_sums(const jg_halo_geom* geom, int dtype) {
+  if (check_geom(geom, "jg_halo_fold_border_takes_sums", true) || (dtype != JG_F32 && dtype != JG_BF16 && dtype != JG_F16)) return 0;
+  return takes_sums(to_geom(geom), dtype) ? 1 : 0;
+}
+
+static int fold_border(void* gx, const void* const strips[27], const jg_halo_geom* geom, int dtype, const jg_conv_reduction* later, void* stream) {
   int rc = check_geom(geom, "jg_halo_fold_border_3d", true);
   if (rc) return rc;
   JG_REQUIRE(gx != nullptr && strips != nullptr, "jg_halo_fold_border_3d: NULL pointer");
@@ -1606,13 +1654,18 @@ extern "C" int jg_halo_fold_border_3d(void* gx, const void* const strips[27],
   Geom g = to_geom(geom);
   const int D = g.n[0], H = g.n[1], W = g.n[2];
   const unsigned long long nrows = (unsigned long long)g.planes * D * H;
-  if (nrows == 0 || W == 0) return JG_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   BorderPlan bp;
   unsigned long long row_items = 0, col_items = 0;
+  if (later != nullptr && (later->dtype != dtype || !takes_sums(g, dtype))) {
+    rc = jg::conv_reduce(*later, s);
+    if (rc) return rc;
+    later = nullptr;
+  }
+  if (nrows == 0 || W == 0) return JG_OK;
   JG_REQUIRE(border_plan(g, &bp, &row_items, &col_items), "jg_halo_fold_border_3d: too many rows (%llu)", nrows);
 #define JG_BORDER(DT)                                                  \
-  JG_REQUIRE(launch_border<DT>(tab, gx, g, bp, row_items, col_items, s), \
+  JG_REQUIRE(launch_border<DT>(tab, gx, g, bp, row_items, col_items, s, later), \
              "jg_halo_fold_border_3d: too many border rows (%llu)", row_items)
   if (dtype == JG_F32) JG_BORDER(JG_F32);
   else if (dtype == JG_BF16) JG_BORDER(JG_BF16);
@@ -1620,6 +1673,17 @@ extern "C" int jg_halo_fold_border_3d(void* gx, const void* const strips[27],
 #undef JG_BORDER
   JG_CHECK_LAUNCH("jg_halo_fold_border_3d");
   return JG_OK;
+}
+
+extern "C" int jg_halo_fold_border_3d(void* gx, const void* const strips[27],
+                                      const jg_halo_geom* geom, int dtype, void* stream) {
+  return fold_border(gx, strips, geom, dtype, nullptr, stream);
+}
+
+extern "C" int jg_halo_fold_border_reduce_3d(void* gx, const void* const strips[27], const jg_halo_geom* geom, int dtype,
+                                             const jg_conv_reduction* later, void* stream) {
+  JG_REQUIRE(later != nullptr, "jg_halo_fold_border_reduce_3d: NULL pointer");
+  return fold_border(gx, strips, geom, dtype, later, stream);
 }
 
 extern "C" int jg_halo_fold_2d(void* gx, const void* gx_aug, const void* const strips[9],

@@ -53,6 +53,12 @@ int64_t count(const Shape& s) {
   return n;
 }
 
+// What `Step.backward` leaves of the weight and bias gradient for `finish`, and the memory it is in.
+struct SumsLeft {
+  jg_conv_reduction sums = {};
+  std::vector<at::Tensor> held;
+};
+
 class Step {
  public:
   // Strips: [(offset, slot, shape), ...] with the leading (batch, channel) entries in the shape.
@@ -63,7 +69,7 @@ class Step {
         elem_(elem_size), code_(code), own_(*reinterpret_cast<const jg_halo_geom*>(own)),
         theirs_(*reinterpret_cast<const jg_halo_geom*>(theirs)), same_(same), desc_(*reinterpret_cast<const jg_conv_desc*>(desc)),
         nbytes_(nbytes), recv_fwd_(strips(recv_fwd)), recv_bwd_(strips(recv_bwd)), send_fwd_(strips(send_fwd)),
-        send_bwd_(strips(send_bwd)), fold_(try_fold) {}
+        send_bwd_(strips(send_bwd)), beside_(jg_halo_fold_border_takes_sums(&theirs_, code) == 1), fold_(try_fold) {}
 
   bool sends() const { return !send_fwd_.empty(); }
 
@@ -93,9 +99,10 @@ class Step {
     return py::make_tuple(y, x_aug);
   }
 
-  // (input gradient, weight gradient, bias gradient, strips to send, folded) or None. The input gradient is the
+  // (input gradient, weight gradient, bias gradient, strips to send, folded, sums left) or None. The input gradient is the
   // padded one, or with `folded` the own tile's, to which only the neighbours' blocks are still missing. The
-  // bias gradient is None where only the separate kernels cover the layer.
+  // bias gradient is None where only the separate kernels cover the layer. Sums left (None, or for `finish`): what the weight
+  // and bias gradient still miss.
   py::object backward(const at::Tensor& g_any, const at::Tensor& x_aug, const at::Tensor& w_any, bool need_x, bool need_w, bool need_b,
                       uintptr_t stream) {
     if (g_any.sizes() != at::IntArrayRef(y_shape_) || x_aug.sizes() != at::IntArrayRef(padded_) || !x_aug.is_contiguous() ||
@@ -104,16 +111,23 @@ class Step {
     at::AutoDispatchBelowADInplaceOrView below;
     void* const s = reinterpret_cast<void*>(stream);
     const at::Tensor g = g_any.contiguous(), w = w_any.contiguous();
-    py::object gw = py::none(), gb = py::none(), gx = py::none(), send = py::dict();
+    py::object gw = py::none(), gb = py::none(), gx = py::none(), send = py::dict(), left = py::none();
     bool folded = false;
+    SumsLeft later;
     if (need_w) {
       const at::Tensor gw_t = at::empty(w_shape_, g.options());
       const at::Tensor ws = scratch(nbytes_[JG_CONV_WGRAD], g);
       int rc = JG_ERR_UNSUPPORTED;
       if (need_b) {
         const at::Tensor gb_t = at::empty({w_shape_[0]}, g.options());
-        rc = jg_conv_wgrad_bias(gw_t.data_ptr(), gb_t.data_ptr(), x_aug.data_ptr(), g.data_ptr(), &desc_, code_, address(ws),
-                                nbytes_[JG_CONV_WGRAD], s);
+        if (need_x && beside_ && fold_.load(std::memory_order_relaxed)) {  // the last of the sums beside the border cells, in `finish`
+          rc = jg_conv_wgrad_bias_later(&later.sums, gw_t.data_ptr(), gb_t.data_ptr(), x_aug.data_ptr(), g.data_ptr(), &desc_, code_,
+                                        address(ws), nbytes_[JG_CONV_WGRAD], s);
+          later.held = {ws, gw_t, gb_t};
+        } else {
+          rc = jg_conv_wgrad_bias(gw_t.data_ptr(), gb_t.data_ptr(), x_aug.data_ptr(), g.data_ptr(), &desc_, code_, address(ws),
+                                  nbytes_[JG_CONV_WGRAD], s);
+        }
         if (rc != JG_ERR_UNSUPPORTED) {
           check(rc, "jg_conv_wgrad_bias");
           gb = py::cast(gb_t);
@@ -142,6 +156,10 @@ class Step {
           fold_.store(false, std::memory_order_relaxed);
         }
       }
+      if (later.sums.kind != 0) {
+        if (folded) left = py::cast(std::move(later));
+        else check(jg_conv_reduce(&later.sums, s), "jg_conv_reduce");
+      }
       if (!folded) {
         const at::Tensor need = at::empty(padded_, g.options());
         check(jg_conv_dgrad(need.data_ptr(), w.data_ptr(), g.data_ptr(), &desc_, code_, address(ws), nbytes_[JG_CONV_DGRAD], s),
@@ -150,15 +168,19 @@ class Step {
         if (!send_bwd_.empty()) send = cut(need, send_bwd_, own_, 1, stream);
       }
     }
-    return py::make_tuple(gx, gw, gb, send, folded);
+    return py::make_tuple(gx, gw, gb, send, folded, left);
   }
 
-  // The own tile's gradient from what `backward` returned and the neighbours' blocks, or None.
-  py::object finish(const at::Tensor& part, bool folded, const py::object& recv, uintptr_t stream) const {
+  // The own tile's gradient from what `backward` returned and the neighbours' blocks, or None. The sums left are done in any case.
+  py::object finish(const at::Tensor& part, bool folded, const py::object& recv, uintptr_t stream, const py::object& left) const {
     const void* tab[27] = {};
-    if (!table(recv, recv_bwd_, part, tab)) return py::none();
-    at::AutoDispatchBelowADInplaceOrView below;
     void* const s = reinterpret_cast<void*>(stream);
+    const jg_conv_reduction* const sums = left.is_none() ? nullptr : &left.cast<const SumsLeft&>().sums;
+    if (!table(recv, recv_bwd_, part, tab)) {
+      if (sums != nullptr) check(jg_conv_reduce(sums, s), "jg_conv_reduce");
+      return py::none();
+    }
+    at::AutoDispatchBelowADInplaceOrView below;
     at::Tensor gx = part;
     const void* none[27] = {};
     if (!folded) {
@@ -166,7 +188,10 @@ class Step {
       // where the neighbours' blocks are not as wide as the own halos, the own part first and the blocks by their widths
       check(jg_halo_fold_3d(gx.data_ptr(), part.data_ptr(), same_ ? tab : none, &own_, code_, s), "jg_halo_fold_3d");
     }
-    if (folded || !same_) check(jg_halo_fold_border_3d(gx.data_ptr(), tab, &theirs_, code_, s), "jg_halo_fold_border_3d");
+    if (sums != nullptr)
+      check(jg_halo_fold_border_reduce_3d(gx.data_ptr(), tab, &theirs_, code_, sums, s), "jg_halo_fold_border_reduce_3d");
+    else if (folded || !same_)
+      check(jg_halo_fold_border_3d(gx.data_ptr(), tab, &theirs_, code_, s), "jg_halo_fold_border_3d");
     return py::cast(gx);
   }
 
@@ -244,6 +269,7 @@ class Step {
   jg_conv_desc desc_;
   std::vector<size_t> nbytes_;
   std::vector<Strip> recv_fwd_, recv_bwd_, send_fwd_, send_bwd_;
+  bool beside_;  // the border's launch takes the sums that the weight gradient leaves
   std::atomic<bool> fold_;
 };
 
@@ -717,6 +743,7 @@ class SwinPass {
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  py::class_<SumsLeft>(m, "SumsLeft");
   py::class_<Step>(m, "Step")
       .def(py::init<const py::tuple&, const py::tuple&, const py::tuple&, const py::tuple&, int, int, uintptr_t, uintptr_t, bool,
                     uintptr_t, const std::vector<size_t>&, const py::list&, const py::list&, const py::list&, const py::list&, bool>())

@@ -941,3 +941,40 @@ def test_fp32_layers_of_few_channels_are_as_exact_as_their_kernels_in_every_dire
     assert rel_l2(y, torch.nn.functional.conv2d(xd, wd)) < 2e-7
     assert rel_l2(gx, torch.nn.grad.conv2d_input(xd.shape, wd, gd)) < 2e-7
     assert rel_l2(gw, torch.nn.grad.conv2d_weight(xd, wd.shape, gd)) < 1e-7
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n, c_in, c_out, size, mesh", [
+    (2, 32, 32, (40, 72), (2, 2)),      # 36 runs of sums in pieces of four, beside the border
+    (1, 5, 7, (9, 11), (3, 3)),         # a single workgroup's partials, odd rows
+    (2, 64, 64, (40, 70), (2, 2)),      # 144 runs
+    (1, 96, 80, (24, 66), (3, 1)),      # several blocks of channels, no neighbour across W
+    (1, 24, 7, (6, 20, 18), (2, 2, 2)),  # three depth taps
+    (4, 40, 8, (300, 310), (3, 3)),     # a border of more blocks than the chip holds: launches of their own
+])
+def test_sums_left_for_the_border_launch_have_the_bits_of_their_own(n, c_in, c_out, size, mesh, dtype, dev):
+    """Weight and bias gradient of the halo convolution, whose last sums run beside the border cells, == conv_nd_weight's."""
+    ns, gen = len(size), torch.Generator().manual_seed(5)
+    k, ones = (3,) * ns, (1,) * ns
+    rank = tuple(1 if m == 3 else 0 for m in mesh)
+    geom = conv_geometry(size, mesh, rank, k, ones, ones, ones)
+    rand = lambda *shape: torch.randn(*shape, generator=gen).to(dtype).to(dev)  # noqa: E731
+    lead = (n, c_in)
+    present = [o for o in geom.offsets() if all(v == 0 or 0 <= r + v < m for v, r, m in zip(o, rank, mesh))]
+    recv_f = {o: rand(*lead, *geom.strip_extent(o, "assemble")) for o in present}
+    recv_b = {o: rand(*lead, *geom.strip_extent(o, "fold")) for o in present}
+    w, b = rand(c_out, c_in, *k).div_(8), rand(c_out)
+    cfg = jc.HipConvNdConfig.for_rank(ns, b, TableExchange(recv_f, recv_b))
+    groups = tuple(jc.TileGroup(m, r) for m, r in zip(mesh, rank))
+    x, wl, bl = rand(*lead, *size).requires_grad_(), w.clone().requires_grad_(), b.clone().requires_grad_()
+    y, x_aug = jc._ConvNd.apply(x, wl, bl, ones, ones, ones, groups, None, cfg)
+    g = rand(*y.shape)
+    gx, gw, gb = torch.autograd.grad(y, (x, wl, bl), g)
+    lp = oh.local_padding(ones, mesh)
+    want_w, want_b = jc.conv_nd_weight(x_aug, w.shape, g, padding=lp, with_bias_grad=True)
+    assert torch.equal(gw, want_w) and torch.equal(gb, want_b)
+    need = jc.conv_nd_input(x_aug.shape, w, g, padding=lp)
+    from jigsaw_amd.halo import halo_fold
+
+    assert torch.equal(gx, halo_fold(need, recv_b, geom))
