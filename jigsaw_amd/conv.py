@@ -937,9 +937,8 @@ class HaloExchange(Protocol):
 
 
 def _mesh_position(spatial_groups) -> tuple[tuple, tuple]:
-    sizes = tuple(1 if g is None else int(g.size()) for g in spatial_groups)
-    ranks = tuple(0 if g is None else int(g.rank()) for g in spatial_groups)
-    return ranks, sizes
+    # (lists: on the way of every step, where generators cost 2 us more of the host)
+    return tuple([0 if g is None else int(g.rank()) for g in spatial_groups]), tuple([1 if g is None else int(g.size()) for g in spatial_groups])
 
 
 @lru_cache(maxsize=256)
@@ -1084,12 +1083,11 @@ def conv_halo_nway_backward(
     """
     n = config.n_spatial
     ranks, sizes = _mesh_position(spatial_groups)
-    local_padding = _local_padding(padding, sizes)
     need_x, need_w = need[0], need[1]
     # a third entry asks for the bias gradient too; the result then has three entries
     want_b = len(need) > 2
     need_b = want_b and need[2]
-    g = grad_output.to(weight.dtype)
+    g = grad_output if grad_output.dtype == weight.dtype else grad_output.to(weight.dtype)
     done = (lambda gx: (gx, g_w, g_b)) if want_b else (lambda gx: (gx, g_w))
     g_w = g_b = None
     if x_tile is None and g.is_cuda and x_aug.dtype == g.dtype and not getattr(x_aug, "_jg_frame_only", False):
@@ -1108,6 +1106,7 @@ def conv_halo_nway_backward(
                 geom = HaloGeometry.for_conv(local_in_spatial, weight.shape[-n:], stride, padding, dilation, ranks, sizes)
                 g_x = halo_fold_border_(part, recv, geom) if folded else halo_fold(part, recv, geom)
             return done(g_x)
+    local_padding = _local_padding(padding, sizes)
     kwargs = {"stride": stride, "padding": local_padding, "dilation": dilation, "groups": int(getattr(config, "groups_local", 1))}
     if x_tile is None and need_w and getattr(config, "framed", False) and getattr(x_aug, "_jg_frame_only", False):
         raise RuntimeError(
@@ -1351,7 +1350,8 @@ class _ConvNd(PositionalFunction):
                 x_tile = None
         else:
             (x_aug, weight), x_tile = ctx.saved_tensors, None
-        x_aug = x_aug.to(weight.dtype)
+        if x_aug.dtype != weight.dtype:
+            x_aug = x_aug.to(weight.dtype)
         need_x, need_w, need_b = ctx.needs_input_grad[:3]
         need_b = need_b and ctx.has_bias
         if getattr(config, "fused_bias_grad", False):
