@@ -36,8 +36,8 @@ constexpr int IN_ROWS = TH + 2, IN_COLS = TW + 2;
 constexpr int PITCH = 68, PLANE = 720;                 // floats of a row and of a channel's window in LDS
 constexpr int CK = 8;                                  // channels of a stage
 constexpr int X_ROWS = CK * IN_ROWS;                   // 80
-constexpr int ROWS_PER_WAVE = X_ROWS / WAVES;          // 20
-static_assert(IN_ROWS * PITCH <= PLANE && PLANE % 64 == 16 && X_ROWS % WAVES == 0 && X_ROWS * 2 <= THREADS, "staging layout");
+constexpr int CH_PER_WAVE = CK / WAVES;                // 2
+static_assert(IN_ROWS * PITCH <= PLANE && PLANE % 64 == 16 && CK % WAVES == 0 && X_ROWS * 2 <= THREADS, "staging layout");
 
 struct Strips {
   void* p[27];
@@ -59,9 +59,15 @@ enum Out { OUT_ROWS, OUT_STREAM, OUT_FOLD };
 
 // SUMS: more than one stage; what a stage adds up goes to a second set of accumulators, so that no sum is longer than a stage's 72
 // products and the number of stages.
+// MT == 0: four produced channels, on v_mfma_f32_4x4x1_16b_f32, whose sixteen blocks are 64 pixels of a row times one channel of one tap: the
+// 16 x 16 products waste the rows of the channels that do not exist, and with 3 of 16 they were 11 of the kernel's 28 us. A
+// lane owns a pixel; the three tap rows have chains of their own (24 products each; relative error of 16 -> 3 channels 1.9e-7 -> 1.2e-7).
+// Input gradient of 4 x 3 -> 16, 256^2 31.6 -> 13.4 us (with the staging below), forward of 2 x 60 -> 4, 200 x 100 46.0 -> 20.4.
 template <int MT, Out OUT, bool SUMS>
-__global__ __launch_bounds__(THREADS, MT == 2 ? 2 : (SUMS ? 3 : 4)) void conv_f32_kernel(Strips strips, Params p) {
-  constexpr int W_FLOATS = CK * 9 * MT * 16;
+__global__ __launch_bounds__(THREADS, MT == 2 ? 2 : (SUMS && MT != 0 ? 3 : 4)) void conv_f32_kernel(Strips strips, Params p) {
+  constexpr bool FEW = MT == 0;
+  constexpr int MC = FEW ? 4 : MT * 16;  // produced channels of a workgroup
+  constexpr int W_FLOATS = CK * 9 * MC;
   __shared__ float lds_x[CK * PLANE];
   __shared__ float lds_w[W_FLOATS];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -69,7 +75,7 @@ __global__ __launch_bounds__(THREADS, MT == 2 ? 2 : (SUMS ? 3 : 4)) void conv_f3
   const int per_image = p.tiles_h * p.tiles_w;
   const int n = blockIdx.x / per_image, t = blockIdx.x - n * per_image;
   const int th = t / p.tiles_w, tw = t - th * p.tiles_w;
-  const int m0 = blockIdx.y * MT * 16;
+  const int m0 = blockIdx.y * MC;
   const int y0 = th * TH - p.pad_h, x0 = tw * TW - p.pad_w;  // window origin
   const size_t plane = (size_t)p.H * p.W;
   const float* image = p.x + (size_t)n * p.C * plane;
@@ -81,78 +87,127 @@ __global__ __launch_bounds__(THREADS, MT == 2 ? 2 : (SUMS ? 3 : 4)) void conv_f3
   const int tail_row = min(tid >> 1, X_ROWS - 1), tail_col = TW + (tid & 1);
   const int tx = x0 + tail_col, txc = min(max(tx, 0), p.W - 1), ty = y0 + tail_row % IN_ROWS;
   const bool tail_ok = tid < 2 * X_ROWS && tx >= 0 && tx < p.W && ty >= 0 && ty < p.H;
-  float xr[ROWS_PER_WAVE], xt = 0.0f;
-  auto row_of = [&](int i, int c0, int* c, int* gy) {  // row i of the wavefront: i * 4 + wave of the stage
-    const int r = i * WAVES + wave;
-    *c = c0 + r / IN_ROWS;
-    *gy = y0 + r % IN_ROWS;
-    return *c < p.C && *gy >= 0 && *gy < p.H;
-  };
+  // A wavefront's rows are those of two channels of the stage: the places in LDS are constants, the two channels share their rows' offsets and
+  // masks. (Rows dealt to the wavefronts in turn took a product and a test for each of twenty, twice a stage, and over 150 scalar
+  // registers in spills: 3 -> 16 of 4 x 256^2 forward 12.3 -> 9.6 us, 16 -> 16 of 8 x 256^2 48.6 -> 40.6 and 58.8 -> 48.5 its gradient, 80 -> 6
+  // of 2 x 256^2 86 -> 65.)
+  float xr[CH_PER_WAVE][IN_ROWS], xt = 0.0f;
   auto issue = [&](int c0) {
+    const float* chan[CH_PER_WAVE];
 #pragma unroll
-    for (int i = 0; i < ROWS_PER_WAVE; ++i) {
-      int c, gy;
-      const bool ok = row_of(i, c0, &c, &gy);
-      xr[i] = image[(ok ? (size_t)c * plane + (size_t)gy * p.W : 0) + gxc];
+    for (int j = 0; j < CH_PER_WAVE; ++j) chan[j] = image + (size_t)min(c0 + wave * CH_PER_WAVE + j, p.C - 1) * plane;
+#pragma unroll
+    for (int r = 0; r < IN_ROWS; ++r) {
+      const uint32_t off = (uint32_t)(min(max(y0 + r, 0), p.H - 1) * p.W + gxc);
+#pragma unroll
+      for (int j = 0; j < CH_PER_WAVE; ++j) xr[j][r] = chan[j][off];
     }
     const int c = c0 + tail_row / IN_ROWS;
     xt = image[(tail_ok && c < p.C ? (size_t)c * plane + (size_t)ty * p.W : 0) + txc];
   };
   auto store = [&](int c0) {
+    float* const to = lds_x + wave * (CH_PER_WAVE * PLANE) + lane;
 #pragma unroll
-    for (int i = 0; i < ROWS_PER_WAVE; ++i) {
-      int c, gy;
-      const bool ok = row_of(i, c0, &c, &gy);
-      const int r = i * WAVES + wave;
-      lds_x[r / IN_ROWS * PLANE + r % IN_ROWS * PITCH + lane] = ok && col_ok ? xr[i] : 0.0f;
+    for (int r = 0; r < IN_ROWS; ++r) {
+      const bool row_ok = col_ok && y0 + r >= 0 && y0 + r < p.H;
+#pragma unroll
+      for (int j = 0; j < CH_PER_WAVE; ++j) to[j * PLANE + r * PITCH] = row_ok && c0 + wave * CH_PER_WAVE + j < p.C ? xr[j][r] : 0.0f;
     }
     if (tid < 2 * X_ROWS)
       lds_x[tail_row / IN_ROWS * PLANE + tail_row % IN_ROWS * PITCH + tail_col] = tail_ok && c0 + tail_row / IN_ROWS < p.C ? xt : 0.0f;
   };
-  // weights of a stage: [tap][four channels][channel of the four][16 MT produced channels]
+  // Weights of a stage, [tap][channel][produced channels] in LDS. Fetched where they are stored; with 32 produced channels and several
+  // stages on their way in registers beside the window's rows (14 -> 45 of 7 x 70 x 313 54.4 -> 51.5 us, 40 -> 24 of 2 x 100^2 37.1 -> 33.9): the others
+  // spill or lose a wavefront's registers by it (3 -> 16 of 4 x 256^2 9.6 -> 12.3, 6 -> 80 of 2 x 256^2 26.5 -> 32.1).
+  constexpr bool AHEAD = MT == 2 && SUMS;
+  constexpr int W_ROUNDS = (W_FLOATS + THREADS - 1) / THREADS;
+  float wr[W_ROUNDS];
+  auto issue_weights = [&](int c0) {  // what does not exist is read from the last that does
+#pragma unroll
+    for (int e = 0; e < W_ROUNDS; ++e) {
+      const int i = min(tid + e * THREADS, W_FLOATS - 1), m = min(m0 + i % MC, p.M - 1), k = i / MC, tap = k >> 3, c = min(c0 + (k & 7), p.C - 1);
+      wr[e] = p.w[p.transposed ? ((size_t)c * p.M + m) * 9 + 8 - tap : ((size_t)m * p.C + c) * 9 + tap];
+    }
+  };
+  auto store_weights = [&](int c0) {
+#pragma unroll
+    for (int e = 0; e < W_ROUNDS; ++e) {
+      const int i = tid + e * THREADS;
+      if (W_FLOATS % THREADS == 0 || i < W_FLOATS) lds_w[i] = m0 + i % MC < p.M && c0 + (i / MC & 7) < p.C ? wr[e] : 0.0f;
+    }
+  };
   auto weights = [&](int c0) {
     for (int i = tid; i < W_FLOATS; i += THREADS) {
-      const int m = m0 + i % (MT * 16), k = i / (MT * 16), tap = k >> 3, c = c0 + (k & 7);
+      const int m = m0 + i % MC, k = i / MC, tap = k >> 3, c = c0 + (k & 7);
       float v = 0.0f;
       if (m < p.M && c < p.C) v = p.transposed ? p.w[((size_t)c * p.M + m) * 9 + 8 - tap] : p.w[((size_t)m * p.C + c) * 9 + tap];
       lds_w[i] = v;
     }
   };
 
-  f32x4 acc[MT][8], sum[SUMS ? MT : 1][8];
+  f32x4 acc[FEW ? 1 : MT][8], sum[SUMS && !FEW ? MT : 1][8];  // FEW: [row of the wavefront * 3 + tap row], sum [row]
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
+  for (int mt = 0; mt < (FEW ? 1 : MT); ++mt) {
     f32x4 b = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int m = m0 + mt * 16 + 4 * kq + i;
+      const int m = m0 + (FEW ? 0 : mt * 16 + 4 * kq) + i;
       if (p.bias != nullptr && m < p.M) b[i] = p.bias[m];
     }
 #pragma unroll
     for (int nb = 0; nb < 8; ++nb) {
-      acc[mt][nb] = b;
+      acc[mt][nb] = FEW && nb % 3 != 0 ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : b;
       if (SUMS) sum[mt][nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
   }
   const bool live = th * TH + wave * 2 < p.Ho;
-  const float* const xb = lds_x + kq * PLANE + wave * 2 * PITCH + n16;
-  const float* const wb = lds_w + kq * (MT * 16) + n16;
+  const float* const xb = FEW ? lds_x + wave * 2 * PITCH + lane : lds_x + kq * PLANE + wave * 2 * PITCH + n16;
+  const float* const wb = FEW ? lds_w + (lane & 3) : lds_w + kq * MC + n16;
   issue(0);
+  if (AHEAD) issue_weights(0);
   for (int c0 = 0; c0 < p.C; c0 += CK) {
     if (c0 > 0) __syncthreads();
     store(c0);
-    weights(c0);
+    if (AHEAD) store_weights(c0);
+    else weights(c0);
     __syncthreads();
-    if (c0 + CK < p.C) issue(c0 + CK);
+    if (c0 + CK < p.C) {
+      issue(c0 + CK);
+      if (AHEAD) issue_weights(c0 + CK);
+    }
     if (!live) continue;
+    if constexpr (FEW) {
+#pragma unroll 2
+      for (int c = 0; c < CK && c0 + c < p.C; ++c) {
+        float a[9], b[4][3];
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap) a[tap] = wb[(tap * CK + c) * MC];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int kw = 0; kw < 3; ++kw) b[r][kw] = xb[c * PLANE + r * PITCH + kw];
+#pragma unroll
+        for (int kw = 0; kw < 3; ++kw)
+#pragma unroll
+          for (int q = 0; q < 6; ++q)
+            acc[0][q] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[q % 3 * 3 + kw], b[q / 3 + q % 3][kw], acc[0][q], 0, 0, 0);
+      }
+      if (SUMS) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) sum[0][r] += (acc[0][3 * r] + acc[0][3 * r + 1]) + acc[0][3 * r + 2];
+#pragma unroll
+        for (int q = 0; q < 6; ++q) acc[0][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+      continue;
+    }
     for (int cg = 0; cg < 2 && c0 + cg * 4 < p.C; ++cg) {
       const float* const xg = xb + cg * 4 * PLANE;
-      const float* const wg = wb + cg * 4 * (MT * 16);
+      const float* const wg = wb + cg * 4 * MC;
 #pragma unroll
       for (int tap = 0; tap < 9; ++tap) {
-        float a[MT];
+        float a[FEW ? 1 : MT];
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) a[mt] = wg[tap * 8 * (MT * 16) + mt * 16];
+        for (int mt = 0; mt < MT; ++mt) a[mt] = wg[tap * 8 * MC + mt * 16];
 #pragma unroll
         for (int nb = 0; nb < 8; ++nb) {
           const float b = xg[(nb / 4 + tap / 3) * PITCH + nb % 4 * 16 + tap % 3];
@@ -173,11 +228,12 @@ __global__ __launch_bounds__(THREADS, MT == 2 ? 2 : (SUMS ? 3 : 4)) void conv_f3
   }
   if (!live) return;
 
-  // lane (n16, kq), register i of block (mt, nb): channel m0 + 16 mt + 4 kq + i, pixel 16 (nb % 4) + n16 of row nb / 4
+  // lane (n16, kq), register i of block (mt, nb): channel m0 + 16 mt + 4 kq + i, pixel 16 (nb % 4) + n16 of row nb / 4. FEW: register i of
+  // row nb is channel m0 + i of pixel `lane`
   auto region = [](int at, int lo, int size) { return at < lo ? 0 : (at < lo + size ? 1 : 2); };
 #pragma unroll
-  for (int nb = 0; nb < 8; ++nb) {
-    const int oh = th * TH + wave * 2 + nb / 4, ow = tw * TW + nb % 4 * 16 + n16;
+  for (int nb = 0; nb < (FEW ? 2 : 8); ++nb) {
+    const int oh = th * TH + wave * 2 + (FEW ? nb : nb / 4), ow = tw * TW + (FEW ? lane : nb % 4 * 16 + n16);
     if (oh >= p.Ho || ow >= p.Wo) continue;
     float* to = p.y;
     int eh = p.Ho, ew = p.Wo, ch = oh, cw = ow;
@@ -195,14 +251,15 @@ __global__ __launch_bounds__(THREADS, MT == 2 ? 2 : (SUMS ? 3 : 4)) void conv_f3
       if (to == nullptr) continue;
     }
     const size_t step = (size_t)eh * ew;
-    float* at = to + ((size_t)n * p.M + m0 + 4 * kq) * step + (size_t)ch * ew + cw;
+    const int mq = FEW ? m0 : m0 + 4 * kq;
+    float* at = to + ((size_t)n * p.M + mq) * step + (size_t)ch * ew + cw;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int mt = 0; mt < (FEW ? 1 : MT); ++mt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        if (m0 + mt * 16 + 4 * kq + i >= p.M) continue;
+        if (mq + mt * 16 + i >= p.M) continue;
         // (`0 + v`: with a fold the sign of a zero is cleared, as the reference's scatter-add does)
-        const float v = SUMS ? sum[mt][nb][i] : acc[mt][nb][i];
+        const float v = SUMS ? sum[mt][nb][i] : FEW ? (acc[0][3 * nb % 8][i] + acc[0][(3 * nb + 1) % 8][i]) + acc[0][(3 * nb + 2) % 8][i] : acc[mt][nb][i];
         if (OUT == OUT_STREAM) __builtin_nontemporal_store(v, at + (mt * 16 + i) * step);
         else at[(mt * 16 + i) * step] = OUT == OUT_FOLD ? v + 0.0f : v;
       }
@@ -381,12 +438,12 @@ bool aligned4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3) == 0;
 int launch(Params p, const Strips& strips, bool fold, hipStream_t s, const char* who) {
   p.tiles_h = (p.Ho + TH - 1) / TH;
   p.tiles_w = (p.Wo + TW - 1) / TW;
-  const int MT = p.M > 16 ? 2 : 1;
-  const dim3 grid((unsigned)(p.N * p.tiles_h * p.tiles_w), (unsigned)((p.M + MT * 16 - 1) / (MT * 16)));
+  const int MT = p.M > 16 ? 2 : p.M > 4 ? 1 : 0, MC = MT == 0 ? 4 : MT * 16;
+  const dim3 grid((unsigned)(p.N * p.tiles_h * p.tiles_w), (unsigned)((p.M + MC - 1) / MC));
   auto pick = [&](auto out_c) -> void (*)(Strips, Params) {
     constexpr Out O = decltype(out_c)::value;
-    if (p.C > CK) return MT == 2 ? &conv_f32_kernel<2, O, true> : &conv_f32_kernel<1, O, true>;
-    return MT == 2 ? &conv_f32_kernel<2, O, false> : &conv_f32_kernel<1, O, false>;
+    if (p.C > CK) return MT == 2 ? &conv_f32_kernel<2, O, true> : MT == 1 ? &conv_f32_kernel<1, O, true> : &conv_f32_kernel<0, O, true>;
+    return MT == 2 ? &conv_f32_kernel<2, O, false> : MT == 1 ? &conv_f32_kernel<1, O, false> : &conv_f32_kernel<0, O, false>;
   };
   void (*kern)(Strips, Params) = nullptr;
   if (fold) kern = pick(std::integral_constant<Out, OUT_FOLD>{});

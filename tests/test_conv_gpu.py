@@ -978,3 +978,19 @@ def test_sums_left_for_the_border_launch_have_the_bits_of_their_own(n, c_in, c_o
     from jigsaw_amd.halo import halo_fold
 
     assert torch.equal(gx, halo_fold(need, recv_b, geom))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c_in, c_out, size", [
+    (1, 1, (1, 1)), (3, 4, (8, 64)), (8, 3, (9, 65)), (9, 4, (17, 130)), (16, 5, (7, 63)), (17, 2, (30, 66)), (5, 33, (12, 70)), (20, 24, (25, 67)),
+])
+def test_fp32_layers_of_few_channels_at_the_edges_of_tiles(c_in, c_out, size, dev):
+    """Four produced channels and fewer have products of their own (conv_f32.hip); stages of eight channels, tiles of 8 x 64."""
+    torch.manual_seed(3)
+    x, w, b = torch.randn(2, c_in, *size), torch.randn(c_out, c_in, 3, 3) / (9 * c_in) ** 0.5, torch.randn(c_out)
+    g = torch.randn(2, c_out, *size)
+    y = jc.conv_nd(x.to(dev), w.to(dev), b.to(dev), padding=1)
+    gx = jc.conv_nd_input(x.shape, w.to(dev), g.to(dev), padding=1)
+    # sums of at most 300 fp32 products: a relative error of 1e-6 is several times what their rounding leaves
+    assert rel_l2(y, torch.nn.functional.conv2d(x.double(), w.double(), b.double(), padding=1)) < 1e-6
+    assert rel_l2(gx, torch.nn.functional.conv_transpose2d(g.double(), w.double(), padding=1)) < 1e-6
