@@ -49,6 +49,7 @@ struct Params {
   const float* bias;
   float* y;        // (N, M, Ho, Wo), or with a fold the tile (N, M, nH, nW)
   int N, C, M, H, W, Ho, Wo, pad_h, pad_w, tiles_h, tiles_w;
+  jg::Div by_image, by_tw;  // tiles of an image, tile columns
   int transposed;
   int lo_h, lo_w, nH, nW;
 };
@@ -73,8 +74,8 @@ __global__ __launch_bounds__(THREADS, MT == 2 ? 2 : (SUMS && MT != 0 ? 3 : 4)) v
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n16 = lane & 15, kq = lane >> 4;
   const int per_image = p.tiles_h * p.tiles_w;
-  const int n = blockIdx.x / per_image, t = blockIdx.x - n * per_image;
-  const int th = t / p.tiles_w, tw = t - th * p.tiles_w;
+  const int n = jg::quotient(blockIdx.x, p.by_image), t = blockIdx.x - n * per_image;
+  const int th = jg::quotient(t, p.by_tw), tw = t - th * p.tiles_w;
   const int m0 = blockIdx.y * MC;
   const int y0 = th * TH - p.pad_h, x0 = tw * TW - p.pad_w;  // window origin
   const size_t plane = (size_t)p.H * p.W;
@@ -278,6 +279,7 @@ struct WgradParams {
   float* part;  // [block][slot][16 MT][columns]
   int N, C, M, H, W, Ho, Wo, pad_h, pad_w, tiles_h, tiles_w, ci_blocks;
   int total, per;  // tiles, and how many a workgroup takes
+  jg::Div by_image, by_tw, by_ci;  // tiles of an image, tile columns, blocks of input channels
 };
 
 // NB blocks of 16 columns a wavefront, the rows of a tile split over RS groups of wavefronts. CI input channels: as many as
@@ -285,38 +287,50 @@ struct WgradParams {
 template <int MT, int NB, int RS>
 __global__ __launch_bounds__(THREADS) void wgrad_f32_kernel(WgradParams p) {
   constexpr int NW = WAVES / RS, COLS = NW * NB * 16, CI = (COLS - 1) / 9;
-  constexpr int XROWS = CI * GX_ROWS, GROWS = MT * 16 * GR;
-  constexpr int XPW = (XROWS + WAVES - 1) / WAVES, GPW = GROWS / WAVES, TAILS = (2 * XROWS + THREADS - 1) / THREADS;
+  constexpr int XROWS = CI * GX_ROWS, GPW = MT * 16, TAILS = (2 * XROWS + THREADS - 1) / THREADS;
+  constexpr int CPW = (CI + WAVES - 1) / WAVES;  // input channels of a wavefront
+  static_assert(GR == WAVES, "a wavefront takes one row of every g channel");
   __shared__ float lds_x[CI * GX_PLANE];
   __shared__ float lds_g[MT * 16 * G_PLANE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n16 = lane & 15, kq = lane >> 4, wn = wave % NW, rs = wave / NW;
-  const int ci0 = blockIdx.y % p.ci_blocks * CI, co0 = blockIdx.y / p.ci_blocks * (MT * 16);
+  const int co_block = jg::quotient(blockIdx.y, p.by_ci);
+  const int ci0 = ((int)blockIdx.y - co_block * p.ci_blocks) * CI, co0 = co_block * (MT * 16);
   const size_t plane_x = (size_t)p.H * p.W, plane_g = (size_t)p.Ho * p.Wo;
   const int begin = min((int)blockIdx.x * p.per, p.total), end = min(begin + p.per, p.total);
 
-  float xr[XPW], gr[GPW], xt[TAILS];
+  // A wavefront fetches the six rows of every fourth input channel and one row of every output channel: its rows' offsets and masks are
+  // shared by the channels, whose addresses walk. (Rows dealt to the wavefronts in turn took a 64-bit product, two clamps and a test each,
+  // 35 to 55 of them twice a tile: 85 to 433 scalar registers in spills. 4 x 3 -> 16, 256^2 13.4 -> 10.5 us, 8 x 16 -> 16, 256^2 89.9 -> 77.4,
+  // 7 x 14 -> 45, 70 x 313 63.4 -> 55.0, 6 x 68 -> 13, 39 x 57 18.0 -> 13.0.)
+  float xr[CPW][GX_ROWS], gr[GPW], xt[TAILS];
   struct At {
     int n, y0, x0, oh0, ow0;
   };
   auto where = [&](int tile) {
-    const int per_image = p.tiles_h * p.tiles_w, n = tile / per_image, t = tile - n * per_image;
-    const int th = t / p.tiles_w, tw = t - th * p.tiles_w;
+    const int per_image = p.tiles_h * p.tiles_w, n = jg::quotient(tile, p.by_image), t = tile - n * per_image;
+    const int th = jg::quotient(t, p.by_tw), tw = t - th * p.tiles_w;
     return At{n, th * GR - p.pad_h, tw * TW - p.pad_w, th * GR, tw * TW};
   };
   auto issue = [&](const At& a) {
     const float* xi = p.x + (size_t)a.n * p.C * plane_x;
     const float* gi = p.g + (size_t)a.n * p.M * plane_g;
     const int gxc = min(max(a.x0 + lane, 0), p.W - 1), owc = min(a.ow0 + lane, p.Wo - 1);
+    uint32_t off[GX_ROWS];
 #pragma unroll
-    for (int i = 0; i < XPW; ++i) {
-      const int r = min(i * WAVES + wave, XROWS - 1), c = min(ci0 + r / GX_ROWS, p.C - 1), y = min(max(a.y0 + r % GX_ROWS, 0), p.H - 1);
-      xr[i] = xi[(size_t)c * plane_x + (size_t)y * p.W + gxc];
+    for (int r = 0; r < GX_ROWS; ++r) off[r] = (uint32_t)(min(max(a.y0 + r, 0), p.H - 1) * p.W + gxc);
+#pragma unroll
+    for (int j = 0; j < CPW; ++j) {
+      const float* const chan = xi + (size_t)min(ci0 + min(j * WAVES + wave, CI - 1), p.C - 1) * plane_x;
+#pragma unroll
+      for (int r = 0; r < GX_ROWS; ++r) xr[j][r] = chan[off[r]];
     }
+    const float* chan = gi + (size_t)co0 * plane_g;
+    const uint32_t at = (uint32_t)(min(a.oh0 + wave, p.Ho - 1) * p.Wo + owc);
 #pragma unroll
     for (int i = 0; i < GPW; ++i) {
-      const int r = i * WAVES + wave, c = min(co0 + r / GR, p.M - 1), y = min(a.oh0 + r % GR, p.Ho - 1);
-      gr[i] = gi[(size_t)c * plane_g + (size_t)y * p.Wo + owc];
+      gr[i] = chan[at];
+      chan += co0 + i + 1 < p.M ? plane_g : 0;
     }
 #pragma unroll
     for (int i = 0; i < TAILS; ++i) {
@@ -327,16 +341,16 @@ __global__ __launch_bounds__(THREADS) void wgrad_f32_kernel(WgradParams p) {
   };
   auto store = [&](const At& a) {
     const bool x_ok = a.x0 + lane >= 0 && a.x0 + lane < p.W, g_ok = a.ow0 + lane < p.Wo;
+    float* const to = lds_x + wave * GX_PLANE + lane;
 #pragma unroll
-    for (int i = 0; i < XPW; ++i) {
-      const int r = i * WAVES + wave, y = a.y0 + r % GX_ROWS;
-      if (r < XROWS) lds_x[r / GX_ROWS * GX_PLANE + r % GX_ROWS * PITCH + lane] = x_ok && y >= 0 && y < p.H ? xr[i] : 0.0f;
-    }
+    for (int j = 0; j < CPW; ++j)
+      if (CI % WAVES == 0 || j + 1 < CPW || j * WAVES + wave < CI) {
 #pragma unroll
-    for (int i = 0; i < GPW; ++i) {
-      const int r = i * WAVES + wave;
-      lds_g[r / GR * G_PLANE + r % GR * TW + lane] = g_ok && a.oh0 + r % GR < p.Ho ? gr[i] : 0.0f;
-    }
+        for (int r = 0; r < GX_ROWS; ++r) to[j * (WAVES * GX_PLANE) + r * PITCH] = x_ok && a.y0 + r >= 0 && a.y0 + r < p.H ? xr[j][r] : 0.0f;
+      }
+    const bool row_ok = g_ok && a.oh0 + wave < p.Ho;
+#pragma unroll
+    for (int i = 0; i < GPW; ++i) lds_g[i * G_PLANE + wave * TW + lane] = row_ok ? gr[i] : 0.0f;
 #pragma unroll
     for (int i = 0; i < TAILS; ++i) {
       const int e = i * THREADS + tid, r = e >> 1, y = a.y0 + r % GX_ROWS, x = a.x0 + TW + (e & 1);
@@ -438,6 +452,8 @@ bool aligned4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3) == 0;
 int launch(Params p, const Strips& strips, bool fold, hipStream_t s, const char* who) {
   p.tiles_h = (p.Ho + TH - 1) / TH;
   p.tiles_w = (p.Wo + TW - 1) / TW;
+  p.by_image = jg::div_by(p.tiles_h * p.tiles_w);
+  p.by_tw = jg::div_by(p.tiles_w);
   const int MT = p.M > 16 ? 2 : p.M > 4 ? 1 : 0, MC = MT == 0 ? 4 : MT * 16;
   const dim3 grid((unsigned)(p.N * p.tiles_h * p.tiles_w), (unsigned)((p.M + MC - 1) / MC));
   auto pick = [&](auto out_c) -> void (*)(Strips, Params) {
@@ -518,6 +534,9 @@ int f32_wgrad(void* gw, void* gb, const void* x, const void* go, const ConvGeom&
   p.N = (int)g.batch; p.C = g.cin; p.M = g.cout; p.H = g.in[1]; p.W = g.in[2]; p.Ho = g.out[1]; p.Wo = g.out[2];
   p.pad_h = g.p[1]; p.pad_w = g.p[2]; p.tiles_h = q.tiles_h; p.tiles_w = q.tiles_w; p.ci_blocks = q.ci_blocks;
   p.total = q.total; p.per = q.per;
+  p.by_image = div_by(q.tiles_h * q.tiles_w);
+  p.by_tw = div_by(q.tiles_w);
+  p.by_ci = div_by(q.ci_blocks);
   const int blocks = q.ci_blocks * q.co_blocks;
   const dim3 grid((unsigned)q.wgs, (unsigned)blocks);
   void (*kern)(WgradParams) = nullptr;
