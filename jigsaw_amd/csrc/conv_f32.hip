@@ -483,8 +483,13 @@ bool f32_conv_supported(const ConvGeom& g, int dtype) {
   if (tiles >= (1ll << 22) || (g.cin + 13) / 14 * ((g.cout + 15) / 16) >= 65536) return false;
   // Against sums of bf16 parts, forward + both gradients, us (this : that). Up to 16 channels on one side:
   //   4 x 3 -> 16, 256^2 60 : 134   8 x 16 -> 16, 512^2 640 : 708   2 x 12 -> 100, 150^2 154 : 252   8 x 3 -> 64, 512^2 920 : 1829
-  // and a layer whose workgroups are fewer than the compute units is bound by its launches:
+  // and a layer whose workgroups are fewer than the compute units is bound by its launches, 6 here and 12 there, and by stages of which
+  // a compute unit has one at a time. With 65 to 128 channels on one side (more have not been
+  // measured) and up to 64 on the other that holds up to three workgroups for four compute units (kernels alone, without the launches' gaps):
   //   2 x 24 -> 24, 200^2 108 : 153   1 x 64 -> 64, 100^2 161 : 225   1 x 64 -> 64, 180^2 204 : 250   2 x 48 -> 48, 150^2 193 : 227
+  //   1 x 17 -> 65, 40^2 98 : 130     8 x 17 -> 80, 64^2 137 : 155    2 x 20 -> 70, 128^2 131 : 155   1 x 40 -> 80, 256 x 128 170 : 196
+  //   2 x 127 -> 40, 48^2 175 : 215   2 x 48 -> 100, 64^2 161 : 189   4 x 40 -> 66, 48 x 90 144 : 192  1 x 64 -> 80, 128^2 172 : 180
+  //   1 x 32 -> 128, 128^2 180 : 181  but 1 x 128 -> 17, 128 x 256 (256 workgroups) 206 : 196, 3 x 80 -> 128, 64^2 236 : 226
   // Beyond, their rate wins:
   //   4 x 20 -> 20, 300^2 249 : 236   2 x 64 -> 64, 180^2 334 : 289   1 x 96 -> 96, 128^2 263 : 243   8 x 64 -> 64, 512^2 6060 : 3851
   // Within the line the parts are faster in one direction or other of large layers: where 9 to 16 channels go into more than 32
@@ -496,7 +501,7 @@ bool f32_conv_supported(const ConvGeom& g, int dtype) {
   // 2.5e-7, gw 6.4e-8 : 2.0e-7, input gradient of 128 from 16 1.6e-7 : 2.5e-7 (3 channels 0.94e-7 : 1.13e-7).
   const int few = std::min(g.cin, g.cout), many = std::max(g.cin, g.cout);
   const long long workgroups = g.batch * ((g.out[1] + TH - 1) / TH) * ((g.out[2] + TW - 1) / TW) * ((many + 31) / 32);
-  return few <= 16 || (many <= 64 && workgroups <= cu_count());
+  return few <= 16 || (many <= 64 && workgroups <= cu_count()) || (few <= 64 && many <= 128 && 4 * workgroups <= 3ll * cu_count());
 }
 
 int f32_fwd(void* y, const void* x, const void* w, const void* bias, const ConvGeom& g, hipStream_t s) {

@@ -994,3 +994,13 @@ def test_fp32_layers_of_few_channels_at_the_edges_of_tiles(c_in, c_out, size, de
     # sums of at most 300 fp32 products: a relative error of 1e-6 is several times what their rounding leaves
     assert rel_l2(y, torch.nn.functional.conv2d(x.double(), w.double(), b.double(), padding=1)) < 1e-6
     assert rel_l2(gx, torch.nn.functional.conv_transpose2d(g.double(), w.double(), padding=1)) < 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [
+    # more than 64 channels on one side and up to 64 on the other, few workgroups: blocks of 32 produced channels and what they leave,
+    # more stages than a patch is held for, several blocks of the weight gradient's columns
+    (1, 17, 65, (10, 66), (0, 0)), (1, 128, 17, (9, 67), (1, 1)), (2, 64, 128, (19, 40), (1, 0)), (1, 97, 64, (8, 64), (2, 2)), (3, 40, 66, (30, 90), (0, 1)),
+], ids=str)
+def test_fp32_layers_of_many_channels_and_few_workgroups(case, dev):
+    test_fp32_on_the_matrix_instruction(case, dev)
