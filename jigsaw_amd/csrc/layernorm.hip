@@ -638,17 +638,92 @@ __global__ __launch_bounds__(kThreads, CH == 1 ? 4 : 1) void ln_plain_bwd_kernel
 
 // ------------------------------------------------- sharded, rows held in registers
 // The four row kernels of the sharded LayerNorm once more, for local widths that fit the register
-// layout of the unsharded kernels (a multiple of 8 columns, at most G * 8 * kPlainChunks): G lanes
+// layout of the unsharded kernels (a multiple of 4 columns, at most G * 8 * kPlainChunks): G lanes
 // share a row, 64 / G rows per wavefront, 16-byte accesses, U rows of a lane group in flight and
 // one pass over the memory. The arithmetic per element is that of the kernels above.
-template <int DT, int CH>
+//
+// HALF: widths of 8 n + 4 columns. Rows start at multiples of four elements and the last octet of a row is half one. 16-bit rows are
+// read and written by the same 16-byte accesses, at addresses of 8 bytes; the half octet reads the four elements in front of it too
+// and moves its own down, so that no access leaves the row. Before, a wavefront walked such a row by itself, four elements a lane, one row
+// in flight, twice for the variance and with accumulators for every column it might have. Bound by memory; partial_fwd / apply /
+// partial_bwd / bwd_apply, us:
+//   262144 x 132 bf16 73 -> 30 / 88 -> 63 / 82 -> 43 / 65 -> 38   30000 x 1540 bf16 39 -> 25 / 61 -> 57 / 122 -> 49 / 55 -> 48
+//   200000 x 76 fp32 52 -> 16 / 54 -> 32 / 48 -> 23 / 42 -> 31    51966 x 652 fp32 41 -> 33 / 80 / 75 -> 68 / 66
+// 8 columns as they lie in memory (16 or 32 bytes), converted later: a kernel can then request the rows of its
+// next round before it turns to the arithmetic of the current one, and the loads stay in the air meanwhile.
+template <int DT, bool HALF>
+struct Raw8 {
+  typedef typename Elem<DT>::T T;
+  static constexpr int PER = 16 / sizeof(T);
+  struct alignas(HALF ? 4 * sizeof(T) : 16) Pack { T v[PER]; };
+  Pack p[kPlainVec / PER];
+};
+template <int DT, bool HALF>
+__device__ __forceinline__ void load8_raw(const typename Elem<DT>::T* base, long long r, long long rows, int c, int cols,
+                                          Raw8<DT, HALF>& out) {
+  typedef typename Raw8<DT, HALF>::Pack Pack;
+  constexpr int PER = Raw8<DT, HALF>::PER, PACKS = kPlainVec / PER;
+  // always an address inside the tensor (row and column clamped): no branch around the load
+  const typename Elem<DT>::T* p = base + (r < rows ? r : rows - 1) * cols;
+  c = c < cols ? c : 0;
+  const bool half = HALF && c + 4 == cols;  // cols >= 12: four elements lie in front
+#pragma unroll
+  for (int h = 0; h < PACKS; ++h) {
+    // 16 bits: the pack that ends with the row; fp32: the first pack again where there is no second
+    const int at = c + (half ? (PACKS == 1 ? -4 : 0) : h * PER);
+    out.p[h] = *reinterpret_cast<const Pack*>(p + at);
+  }
+}
+template <int DT, bool HALF>
+__device__ __forceinline__ void unpack8(const Raw8<DT, HALF>& in, bool ok, int c, int cols, float out[kPlainVec]) {
+  constexpr int PER = Raw8<DT, HALF>::PER;
+  const bool half = HALF && c + 4 == cols;
+#pragma unroll
+  for (int i = 0; i < kPlainVec; ++i) {
+    float v = Elem<DT>::up(in.p[i / PER].v[i % PER]);
+    if (HALF && PER == kPlainVec && i < 4) v = half ? Elem<DT>::up(in.p[0].v[(i + 4) % PER]) : v;
+    out[i] = ok && !(HALF && i >= 4 && half) ? v : 0.0f;
+  }
+}
+
+// 8 columns of a row from an address that is always inside the tensor (row and column clamped), zero
+// where the lane owns nothing: the loads of a wavefront leave back to back, under no branch.
+template <int DT, bool HALF>
+__device__ __forceinline__ void load8_or_zero(const typename Elem<DT>::T* base, long long r, long long rows, int c,
+                                              int cols, float out[kPlainVec]) {
+  Raw8<DT, HALF> raw;
+  load8_raw<DT, HALF>(base, r, rows, c, cols, raw);
+  unpack8<DT, HALF>(raw, r < rows && c < cols, c, cols, out);
+}
+
+template <int DT, bool HALF>
+__device__ __forceinline__ void store8_of(typename Elem<DT>::T* row, int c, int cols, const float in[kPlainVec]) {
+  typedef typename Elem<DT>::T T;
+  constexpr int PER = Raw8<DT, HALF>::PER;
+  if (!HALF || c + kPlainVec <= cols) {
+#pragma unroll
+    for (int h = 0; h < kPlainVec / PER; ++h) {
+      typename Raw8<DT, HALF>::Pack q;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) q.v[i] = Elem<DT>::down(in[h * PER + i]);
+      *reinterpret_cast<typename Raw8<DT, HALF>::Pack*>(row + c + h * PER) = q;
+    }
+  } else {
+    struct alignas(4 * sizeof(T)) Quad { T v[4]; } q;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q.v[i] = Elem<DT>::down(in[i]);
+    *reinterpret_cast<Quad*>(row + c) = q;
+  }
+}
+
+template <int DT, int CH, bool HALF>
 __device__ __forceinline__ void load_params_of(float (&dst)[CH][kPlainVec], const typename Elem<DT>::T* src, int G,
                                                int sl, int cols) {
 #pragma unroll
   for (int k = 0; k < CH; ++k) {
     const int c = (k * G + sl) * kPlainVec;
     if (c < cols && src != nullptr) {
-      load8<DT>(src + c, dst[k]);
+      load8_or_zero<DT, HALF>(src, 0, 1, c, cols, dst[k]);
     } else {
 #pragma unroll
       for (int i = 0; i < kPlainVec; ++i) dst[k][i] = 0.0f;
@@ -656,44 +731,7 @@ __device__ __forceinline__ void load_params_of(float (&dst)[CH][kPlainVec], cons
   }
 }
 
-// 8 columns of a row from an address that is always inside the tensor (row and column clamped), zero
-// where the lane owns nothing: the loads of a wavefront leave back to back, under no branch.
-template <int DT>
-__device__ __forceinline__ void load8_or_zero(const typename Elem<DT>::T* base, long long r, long long rows, int c,
-                                              int cols, float out[kPlainVec]) {
-  const bool ok = r < rows && c < cols;
-  load8<DT>(base + (r < rows ? r : rows - 1) * cols + (c < cols ? c : 0), out);
-#pragma unroll
-  for (int i = 0; i < kPlainVec; ++i) out[i] = ok ? out[i] : 0.0f;
-}
-
-// 8 columns as they lie in memory (16 or 32 bytes), converted later: a kernel can then request the rows of its
-// next round before it turns to the arithmetic of the current one, and the loads stay in the air meanwhile.
-template <int DT>
-struct Raw8 {
-  typedef typename Elem<DT>::T T;
-  static constexpr int PER = 16 / sizeof(T);
-  struct alignas(16) Pack { T v[PER]; };
-  Pack p[kPlainVec / PER];
-};
-template <int DT>
-__device__ __forceinline__ void load8_raw(const typename Elem<DT>::T* base, long long r, long long rows, int c, int cols,
-                                          Raw8<DT>& out) {
-  typedef typename Raw8<DT>::Pack Pack;
-  // always an address inside the tensor (row and column clamped): no branch around the load
-  const typename Elem<DT>::T* p = base + (r < rows ? r : rows - 1) * cols + (c < cols ? c : 0);
-#pragma unroll
-  for (int h = 0; h < kPlainVec / Raw8<DT>::PER; ++h) out.p[h] = *reinterpret_cast<const Pack*>(p + h * Raw8<DT>::PER);
-}
-template <int DT>
-__device__ __forceinline__ void unpack8(const Raw8<DT>& in, bool ok, float out[kPlainVec]) {
-#pragma unroll
-  for (int h = 0; h < kPlainVec / Raw8<DT>::PER; ++h)
-#pragma unroll
-    for (int i = 0; i < Raw8<DT>::PER; ++i) out[h * Raw8<DT>::PER + i] = ok ? Elem<DT>::up(in.p[h].v[i]) : 0.0f;
-}
-
-template <int DT, int CH, int U>
+template <int DT, int CH, int U, bool HALF>
 __global__ __launch_bounds__(kThreads) void ln_partial_fwd_rows_kernel(
     float* __restrict__ mean, float* __restrict__ mean2, float* __restrict__ var,
     const typename Elem<DT>::T* __restrict__ x, long long rows, int cols, int G) {
@@ -704,12 +742,12 @@ __global__ __launch_bounds__(kThreads) void ln_partial_fwd_rows_kernel(
   const long long stride = rpw;
   const long long round_stride = (long long)gridDim.x * kWavesPerBlock * rpw * U;
   long long r0 = ((long long)blockIdx.x * kWavesPerBlock + wave) * rpw * U;
-  Raw8<DT> raw[U][CH];
+  Raw8<DT, HALF> raw[U][CH];
   auto request = [&](long long first) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int k = 0; k < CH; ++k) load8_raw<DT>(x, first + u * stride + sub, rows, (k * G + sl) * kPlainVec, cols, raw[u][k]);
+      for (int k = 0; k < CH; ++k) load8_raw<DT, HALF>(x, first + u * stride + sub, rows, (k * G + sl) * kPlainVec, cols, raw[u][k]);
   };
   if (r0 < rows) request(r0);
   for (; r0 < rows; r0 += round_stride) {
@@ -719,7 +757,7 @@ __global__ __launch_bounds__(kThreads) void ln_partial_fwd_rows_kernel(
     for (int u = 0; u < U; ++u) {
       live[u] = r0 + u * stride + sub < rows;
 #pragma unroll
-      for (int k = 0; k < CH; ++k) unpack8<DT>(raw[u][k], live[u] && (k * G + sl) * kPlainVec < cols, v[u][k]);
+      for (int k = 0; k < CH; ++k) unpack8<DT, HALF>(raw[u][k], live[u] && (k * G + sl) * kPlainVec < cols, (k * G + sl) * kPlainVec, cols, v[u][k]);
     }
     // the rows of the next round are on their way during the sums and shuffles of this one
     if (r0 + round_stride < rows) request(r0 + round_stride);
@@ -743,7 +781,7 @@ __global__ __launch_bounds__(kThreads) void ln_partial_fwd_rows_kernel(
         if ((k * G + sl) * kPlainVec < cols) {
 #pragma unroll
           for (int i = 0; i < kPlainVec; ++i) {
-            const float d = v[u][k][i] - m[u];
+            const float d = HALF && i >= 4 && (k * G + sl) * kPlainVec + 4 == cols ? 0.0f : v[u][k][i] - m[u];
             q += d * d;
           }
         }
@@ -764,7 +802,7 @@ __global__ __launch_bounds__(kThreads) void ln_partial_fwd_rows_kernel(
   }
 }
 
-template <int XDT, int ODT, int CH, int U>
+template <int XDT, int ODT, int CH, int U, bool HALF>
 __global__ __launch_bounds__(kThreads) void ln_apply_rows_kernel(
     typename Elem<ODT>::T* __restrict__ y, typename Elem<ODT>::T* __restrict__ x_hat,
     float* __restrict__ std_out, typename Elem<ODT>::T* __restrict__ var_out,
@@ -777,8 +815,8 @@ __global__ __launch_bounds__(kThreads) void ln_apply_rows_kernel(
   // a wavefront's U row sets of a round lie behind each other in memory (U * rpw consecutive rows)
   const long long stride = rpw, round_stride = (long long)gridDim.x * kWavesPerBlock * rpw * U;
   float wv[CH][kPlainVec], bv[CH][kPlainVec];
-  load_params_of<ODT, CH>(wv, w, G, sl, cols);
-  load_params_of<ODT, CH>(bv, b, G, sl, cols);
+  load_params_of<ODT, CH, HALF>(wv, w, G, sl, cols);
+  load_params_of<ODT, CH, HALF>(bv, b, G, sl, cols);
   for (long long r0 = ((long long)blockIdx.x * kWavesPerBlock + wave) * rpw * U; r0 < rows; r0 += round_stride) {
     float v[U][CH][kPlainVec], m[U], sd[U];
     bool live[U];
@@ -792,7 +830,7 @@ __global__ __launch_bounds__(kThreads) void ln_apply_rows_kernel(
 #pragma unroll
       for (int k = 0; k < CH; ++k) {
         const int c = (k * G + sl) * kPlainVec;
-        load8_or_zero<XDT>(x, r, rows, c, cols, v[u][k]);
+        load8_or_zero<XDT, HALF>(x, r, rows, c, cols, v[u][k]);
       }
     }
 #pragma unroll
@@ -812,8 +850,8 @@ __global__ __launch_bounds__(kThreads) void ln_apply_rows_kernel(
             xh[i] = Elem<ODT>::up(Elem<ODT>::down((v[u][k][i] - m[u]) / s));
             out[i] = wv[k][i] * xh[i] + bv[k][i];
           }
-          if (x_hat != nullptr) store8<ODT>(x_hat + r * cols + c, xh);
-          store8<ODT>(y + r * cols + c, out);
+          if (x_hat != nullptr) store8_of<ODT, HALF>(x_hat + r * cols, c, cols, xh);
+          store8_of<ODT, HALF>(y + r * cols, c, cols, out);
         }
       }
     }
@@ -824,7 +862,7 @@ __global__ __launch_bounds__(kThreads) void ln_apply_rows_kernel(
 // WAVES wavefronts a block (the number of blocks, and with it of partial rows, is bounded by the workspace
 // contract, so more wavefronts per block is how more rows are in flight per CU); a wavefront's U row sets of
 // a round lie behind each other in memory. Dynamic LDS: WAVES * 2 * cols floats.
-template <int DT, int CH, int U, int WAVES>
+template <int DT, int CH, int U, int WAVES, bool HALF>
 __global__ __launch_bounds__(WAVES * kWave) void ln_partial_bwd_rows_kernel(
     float* __restrict__ mean_gxn, float* __restrict__ dot, float* __restrict__ part,
     const typename Elem<DT>::T* __restrict__ g, const typename Elem<DT>::T* __restrict__ x_hat,
@@ -835,7 +873,7 @@ __global__ __launch_bounds__(WAVES * kWave) void ln_partial_bwd_rows_kernel(
   const float inv = 1.0f / (float)cols;
   const long long round_stride = (long long)gridDim.x * WAVES * rpw * U;
   float wv[CH][kPlainVec], agw[CH][kPlainVec], agb[CH][kPlainVec];
-  load_params_of<DT, CH>(wv, w, G, sl, cols);
+  load_params_of<DT, CH, HALF>(wv, w, G, sl, cols);
 #pragma unroll
   for (int k = 0; k < CH; ++k)
 #pragma unroll
@@ -853,8 +891,8 @@ __global__ __launch_bounds__(WAVES * kWave) void ln_partial_bwd_rows_kernel(
 #pragma unroll
       for (int k = 0; k < CH; ++k) {
         const int c = (k * G + sl) * kPlainVec;
-        load8_or_zero<DT>(g, r, rows, c, cols, gv[u][k]);
-        load8_or_zero<DT>(x_hat, r, rows, c, cols, xh[u][k]);
+        load8_or_zero<DT, HALF>(g, r, rows, c, cols, gv[u][k]);
+        load8_or_zero<DT, HALF>(x_hat, r, rows, c, cols, xh[u][k]);
       }
     }
 #pragma unroll
@@ -919,7 +957,7 @@ __global__ __launch_bounds__(WAVES * kWave) void ln_partial_bwd_rows_kernel(
   }
 }
 
-template <int DT, int CH, int U>
+template <int DT, int CH, int U, bool HALF>
 __global__ __launch_bounds__(kThreads) void ln_bwd_apply_rows_kernel(
     typename Elem<DT>::T* __restrict__ gx, const typename Elem<DT>::T* __restrict__ g,
     const typename Elem<DT>::T* __restrict__ x_hat, const typename Elem<DT>::T* __restrict__ w,
@@ -930,7 +968,7 @@ __global__ __launch_bounds__(kThreads) void ln_bwd_apply_rows_kernel(
   // a wavefront's U row sets of a round lie behind each other in memory (U * rpw consecutive rows)
   const long long stride = rpw, round_stride = (long long)gridDim.x * kWavesPerBlock * rpw * U;
   float wv[CH][kPlainVec];
-  load_params_of<DT, CH>(wv, w, G, sl, cols);
+  load_params_of<DT, CH, HALF>(wv, w, G, sl, cols);
   for (long long r0 = ((long long)blockIdx.x * kWavesPerBlock + wave) * rpw * U; r0 < rows; r0 += round_stride) {
     float gv[U][CH][kPlainVec], xh[U][CH][kPlainVec], m[U], dn[U], sd[U];
     bool live[U];
@@ -945,8 +983,8 @@ __global__ __launch_bounds__(kThreads) void ln_bwd_apply_rows_kernel(
 #pragma unroll
       for (int k = 0; k < CH; ++k) {
         const int c = (k * G + sl) * kPlainVec;
-        load8_or_zero<DT>(g, r, rows, c, cols, gv[u][k]);
-        load8_or_zero<DT>(x_hat, r, rows, c, cols, xh[u][k]);
+        load8_or_zero<DT, HALF>(g, r, rows, c, cols, gv[u][k]);
+        load8_or_zero<DT, HALF>(x_hat, r, rows, c, cols, xh[u][k]);
       }
     }
 #pragma unroll
@@ -964,7 +1002,7 @@ __global__ __launch_bounds__(kThreads) void ln_bwd_apply_rows_kernel(
             const float gxn = Elem<DT>::up(Elem<DT>::down(gv[u][k][i] * wv[k][i]));
             out[i] = rs * (gxn - m[u] - xh[u][k][i] * d);
           }
-          store8<DT>(gx + r * cols + c, out);
+          store8_of<DT, HALF>(gx + r * cols, c, cols, out);
         }
       }
     }
@@ -982,6 +1020,26 @@ int plain_chunks(long long cols) {
   return (int)((cols + (long long)G * kPlainVec - 1) / ((long long)G * kPlainVec));
 }
 bool plain_ok(long long cols) { return cols >= kPlainVec && cols % kPlainVec == 0 && plain_chunks(cols) <= kPlainChunks; }
+// The sharded kernels also take rows whose last octet is half one (HALF), in 16 bits from 2^20 elements on, in fp32 from 2^22: below that
+// every launch is 3 to 7 us either way, and the walking kernels' shorter rounds are up to 1 us ahead (2000 x 132 bf16, the four kernels
+// 14.7 : 17.0; 8000 x 252 fp32, partial_bwd 5.6 : 6.6; but 16000 x 68 bf16 27.2 : 19.2 and 4000 x 1028 fp32, the two that read 21.6 : 20.2).
+bool rows_ok(long long rows, long long cols, int dtype) {
+  if (plain_ok(cols)) return true;
+  const long long least = 1ll << (dtype == JG_F32 ? 22 : 20);
+  return cols > kPlainVec && cols % kPlainVec == 4 && plain_chunks(cols) <= kPlainChunks && rows >= least / cols;
+}
+// The two kernels that write rows, where the walking kernel is the better one (it : rows in registers, apply / bwd_apply, us): fp32 rows that
+// give most lanes of a walking wavefront their 16 bytes, which cover whole lines behind each other while an octet a lane touches each line twice:
+//   100000 x 132 31 : 29 / 28 : 27   100000 x 180 35 : 38 / 34 : 35   100000 x 252 55 : 61 / 47 : 58   100000 x 388 87 : 100 / 72 : 93
+//   60000 x 516 75 : 75 / 63 : 70    40000 x 1300 126 : 119 / 108 : 113   4000 x 1028 10.3 : 13.8 / 10.0 : 11.2
+// and the forward's 16-bit rows whose second chunk is less than half full:
+//   60000 x 516 49 : 52   51966 x 652 46 : 49   60000 x 772 66 : 60   100000 x 508 76 : 66
+bool rows_written_ok(long long rows, long long cols, int out_dtype, bool forward) {
+  if (!rows_ok(rows, cols, out_dtype)) return false;
+  if (cols % kPlainVec == 0) return true;
+  if (out_dtype == JG_F32) return cols <= kWave * kVec * 5 / 8;
+  return !(forward && cols > kWave * kPlainVec && cols < kWave * kPlainVec * 3 / 2);
+}
 int plain_blocks(long long rows, long long cols, int most = 1024) {
   const int rpw = kWave / plain_group(cols);
   long long b = (rows + (long long)kWavesPerBlock * rpw - 1) / ((long long)kWavesPerBlock * rpw);  // one row set a wavefront
@@ -1003,6 +1061,15 @@ void with_row_shape(long long cols, F&& f) {
     case 3: f(integral_constant<int, 3>(), integral_constant<int, 1>()); break;
     default: f(integral_constant<int, 4>(), integral_constant<int, 1>()); break;
   }
+}
+
+// and whether the last octet of a row is half one: f(chunks, rows_in_flight, half)
+template <int U1, typename F>
+void with_sharded_row_shape(long long cols, F&& f) {
+  with_row_shape<U1>(cols, [&](auto ch, auto u) {
+    if (cols % kPlainVec == 0) f(ch, u, std::false_type{});
+    else f(ch, u, std::true_type{});
+  });
 }
 
 template <int XDT, int YDT>
@@ -1059,12 +1126,12 @@ extern "C" int jg_ln_partial_fwd2(float* mean, float* mean2, float* var, const v
   if (rows == 0) return JG_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool v = vec_aligned(x, cols, x_dtype);
-  const bool in_regs = plain_ok(cols) && aligned16(x);
+  const bool in_regs = rows_ok(rows, cols, x_dtype) && aligned16(x);
   const int G = in_regs ? plain_group(cols) : 0, blocks = in_regs ? plain_blocks(rows, cols, 8192) : 0;
 #define JG_GO(DT)                                                                                  \
   if (in_regs)                                                                                     \
-    with_row_shape<4>(cols, [&](auto ch, auto u) {                                                 \
-      ln_partial_fwd_rows_kernel<DT, decltype(ch)::value, decltype(u)::value>                      \
+    with_sharded_row_shape<4>(cols, [&](auto ch, auto u, auto half) {                                                 \
+      ln_partial_fwd_rows_kernel<DT, decltype(ch)::value, decltype(u)::value, decltype(half)::value>                      \
           <<<blocks, kThreads, 0, s>>>(mean, mean2, var, static_cast<const Elem<DT>::T*>(x), rows, (int)cols, G); \
     });                                                                                            \
   else                                                                                             \
@@ -1087,10 +1154,10 @@ static void launch_apply(void* y, void* x_hat, float* std_out, void* var_out, co
   const bool vx = vec_aligned(x, cols, XDT);
   const bool vo = vec_aligned(y, cols, ODT) && (x_hat == nullptr || vec_aligned(x_hat, cols, ODT));
   const bool vw = vec_aligned(w, cols, ODT) && (b == nullptr || vec_aligned(b, cols, ODT));
-  if (plain_ok(cols) && aligned16(x) && aligned16(y) && aligned16(x_hat) && aligned16(w) && aligned16(b)) {
+  if (rows_written_ok(rows, cols, ODT, true) && aligned16(x) && aligned16(y) && aligned16(x_hat) && aligned16(w) && aligned16(b)) {
     const int G = plain_group(cols), blocks = plain_blocks(rows, cols, 2048);
-    with_row_shape<2>(cols, [&](auto ch, auto u) {
-      ln_apply_rows_kernel<XDT, ODT, decltype(ch)::value, decltype(u)::value><<<blocks, kThreads, 0, s>>>(
+    with_sharded_row_shape<2>(cols, [&](auto ch, auto u, auto half) {
+      ln_apply_rows_kernel<XDT, ODT, decltype(ch)::value, decltype(u)::value, decltype(half)::value><<<blocks, kThreads, 0, s>>>(
           static_cast<OT*>(y), static_cast<OT*>(x_hat), std_out, static_cast<OT*>(var_out), static_cast<const XT*>(x), mean, var,
           static_cast<const OT*>(w), static_cast<const OT*>(b), rows, (int)cols, eps, G);
     });
@@ -1154,15 +1221,15 @@ static int launch_partial_bwd(float* mean_gxn, float* dot, float* part, const vo
                               const void* x_hat, const void* w, int64_t rows, int64_t cols,
                               bool want_cols, hipStream_t s, int* blocks_used) {
   typedef typename Elem<DT>::T T;
-  if (plain_ok(cols) && aligned16(g) && aligned16(x_hat) && aligned16(w)) {
+  if (rows_ok(rows, cols, DT) && aligned16(g) && aligned16(x_hat) && aligned16(w)) {
     const int G = plain_group(cols);
     const int rpw = kWave / G;
     long long nb = (rows + (long long)kWavesPerBlock * rpw - 1) / ((long long)kWavesPerBlock * rpw);
     const int blocks = (int)(nb > 1024 ? 1024 : nb);  // never more than bwd_blocks(rows)
     *blocks_used = blocks;
     const size_t lds = (size_t)kWavesPerBlock * 2 * cols * sizeof(float);
-    with_row_shape<2>(cols, [&](auto ch, auto u) {
-      ln_partial_bwd_rows_kernel<DT, decltype(ch)::value, decltype(u)::value, kWavesPerBlock>
+    with_sharded_row_shape<2>(cols, [&](auto ch, auto u, auto half) {
+      ln_partial_bwd_rows_kernel<DT, decltype(ch)::value, decltype(u)::value, kWavesPerBlock, decltype(half)::value>
           <<<blocks, kThreads, lds, s>>>(mean_gxn, dot, part, static_cast<const T*>(g), static_cast<const T*>(x_hat),
                                          static_cast<const T*>(w), rows, (int)cols, G, want_cols);
     });
@@ -1303,10 +1370,10 @@ extern "C" int jg_ln_bwd_apply(void* gx, const void* g, const void* x_hat, const
     const bool v = vec_aligned(g, cols, DT) && vec_aligned(x_hat, cols, DT) &&             \
                    vec_aligned(gx, cols, DT);                                              \
     const bool vw = vec_aligned(w, cols, DT);                                              \
-    if (plain_ok(cols) && aligned16(gx) && aligned16(g) && aligned16(x_hat) && aligned16(w)) { \
+    if (rows_written_ok(rows, cols, DT, false) && aligned16(gx) && aligned16(g) && aligned16(x_hat) && aligned16(w)) { \
       const int G = plain_group(cols), blocks = plain_blocks(rows, cols, 2048);                  \
-      with_row_shape<2>(cols, [&](auto ch, auto u) {                                       \
-        ln_bwd_apply_rows_kernel<DT, decltype(ch)::value, decltype(u)::value>              \
+      with_sharded_row_shape<2>(cols, [&](auto ch, auto u, auto half) {                                       \
+        ln_bwd_apply_rows_kernel<DT, decltype(ch)::value, decltype(u)::value, decltype(half)::value>              \
             <<<blocks, kThreads, 0, s>>>(static_cast<T*>(gx), static_cast<const T*>(g),    \
                                          static_cast<const T*>(x_hat), static_cast<const T*>(w), \
                                          mean_gxn, dot_gxn_xhat, std, rows, (int)cols, inv_n, G); \

@@ -140,6 +140,33 @@ def test_layernorm_two_shards_over_widths(cols, lead, dtype, dev):
             assert got.dtype == dtype and rel_l2(got, want) < 2e-2
 
 
+@pytest.mark.parametrize("cols,dtype", [
+    # rows of 8 n + 4 columns, whose last octet is half one, from 2^20 elements on (fp32 2^22): one to four chunks a lane, the half octet in a row's
+    # first chunk and in its last, alone in a chunk; fp32 rows past 160 columns are written by the kernels that walk a row
+    (12, torch.bfloat16), (12, torch.float32), (20, torch.float16), (132, torch.bfloat16), (252, torch.float32), (260, torch.float32),
+    (516, torch.bfloat16), (652, torch.float32), (772, torch.bfloat16), (1028, torch.float16), (1540, torch.float32), (2044, torch.bfloat16),
+], ids=lambda v: str(v).replace("torch.", ""))
+def test_layernorm_rows_that_end_in_half_an_octet(cols, dtype, dev):
+    lead = ((1 << (22 if dtype == torch.float32 else 20)) // cols + 3,)
+    test_layernorm_two_shards_over_widths(cols, lead, dtype, dev)
+    x = (torch.randn(*lead, cols) * 3 + 1.5).to(dtype)
+    m, v = jl.partial_stats(x.to(dev))
+    wm, wv = ol.partial_stats(x.double())
+    torch.testing.assert_close(m.cpu().double(), wm, atol=1e-5, rtol=1e-5)
+    torch.testing.assert_close(v.cpu().double(), wv, atol=1e-5, rtol=1e-5)
+    # nothing is written past the last row
+    from jigsaw_amd import _lib
+
+    guard = torch.full((x.numel() + 64,), 7.0, dtype=dtype, device=dev)
+    xd, ones = x.to(dev), torch.ones(cols, dtype=dtype, device=dev)
+    rc = _lib.load().jg_ln_apply(_lib.ptr(guard), None, None, _lib.ptr(xd), _lib.ptr(m), _lib.ptr(v), _lib.ptr(ones), None, x.numel() // cols, cols,
+                                 1e-5, _lib.dtype_code(dtype), _lib.dtype_code(dtype), _lib.stream_ptr(dev))
+    _lib.check(rc, "jg_ln_apply")
+    # two roundings, of 2^-9 at most in bf16
+    assert rel_l2(guard[:x.numel()].view(x.shape), F.layer_norm(x.double(), (cols,))) < (1e-5 if dtype == torch.float32 else 4e-3)
+    assert (guard[x.numel():] == 7).all()
+
+
 def test_layernorm_under_autocast_returns_fp32_and_leaf_dtype_grad(dev):
     """LayerNorm under autocast computes in fp32 (reference: tests/test_autocast.py:265-292)."""
     torch.manual_seed(2)
