@@ -15,8 +15,8 @@
 //
 // Beside it, fp32 layers run as sums of three bf16 parts (conv_mfma.hip): a sixth of the bf16 rate, 0.4 PFLOP/s on paper against
 // the 0.16 PFLOP/s of this instruction, but the parts are written and read, in launches of their own, and a step there is 16 channels of
-// six products whatever the layer has. Batch 4, 3 -> 16 channels, 256^2 (that : this): forward 28 : 12 us, both gradients of the
-// weight and bias 46 : 20, input gradient 55 : 28, 14 launches : 7. What bounds it there: latency, at one or two stages a workgroup;
+// six products whatever the layer has. Batch 4, 3 -> 16 channels, 256^2 (that : this): forward 28 : 9.5 us, gradients of the
+// weight and bias 46 : 10.5 and their sums beside the border cells, input gradient 55 : 13, 14 launches : 6. What bounds it there: latency, at one or two stages a workgroup;
 // with many channels the instruction's rate, 74 of 157 TFLOP/s at 20 -> 20 channels, 8 x 500^2. f32_conv_supported has the line
 // between the two. Against float64 no result is further off than the three parts' (relative, 16 channels: y 1.9e-7 : 2.5e-7).
 #include "conv_common.h"
@@ -491,12 +491,13 @@ bool f32_conv_supported(const ConvGeom& g, int dtype) {
   //   2 x 127 -> 40, 48^2 175 : 215   2 x 48 -> 100, 64^2 161 : 189   4 x 40 -> 66, 48 x 90 144 : 192  1 x 64 -> 80, 128^2 172 : 180
   //   1 x 32 -> 128, 128^2 180 : 181  but 1 x 128 -> 17, 128 x 256 (256 workgroups) 206 : 196, 3 x 80 -> 128, 64^2 236 : 226
   // Beyond, their rate wins:
-  //   4 x 20 -> 20, 300^2 249 : 236   2 x 64 -> 64, 180^2 334 : 289   1 x 96 -> 96, 128^2 263 : 243   8 x 64 -> 64, 512^2 6060 : 3851
+  //   4 x 32 -> 32, 256^2 298 : 231   2 x 64 -> 64, 180^2 312 : 228   1 x 96 -> 96, 128^2 229 : 220   8 x 64 -> 64, 512^2 6060 : 3851
+  //   4 x 17 -> 64, 256^2 367 : 313   8 x 20 -> 20, 500^2 1123 : 1074  but 4 x 20 -> 20, 300^2 248 : 259   8 x 28 -> 31, 300^2 553 : 593
   // Within the line the parts are faster in one direction or other of large layers: where 9 to 16 channels go into more than 32
   // (16 fill the parts' step; this has two stages of 8 and half of its rate), and in the weight gradient of 15 to 21 input channels, which need a
-  // second block of columns here (forward, weight gradient, input gradient):
+  // second block of columns here (forward, weight gradient, input gradient; all but the last with staging since made 5 to 20 % faster here):
   //   8 x 16 -> 128, 256^2 242 : 168, 524 : 509, 342 : 418   8 x 128 -> 16, 256^2 301 : 365, 409 : 491, 305 : 224
-  //   4 x 15 -> 18, 512^2 124 : 111, 287 : 151, 117 : 163    8 x 16 -> 16, 256^2 51 : 66, 91 : 88, 54 : 76
+  //   4 x 15 -> 18, 512^2 124 : 111, 287 : 151, 117 : 163    8 x 16 -> 16, 256^2 41 : 66, 77 : 88, 49 : 76
   // Those directions stay here too: the parts are less exact in all of them. Relative error against float64, 16 -> 128: y 1.6e-7 :
   // 2.5e-7, gw 6.4e-8 : 2.0e-7, input gradient of 128 from 16 1.6e-7 : 2.5e-7 (3 channels 0.94e-7 : 1.13e-7).
   const int few = std::min(g.cin, g.cout), many = std::max(g.cin, g.cout);
