@@ -58,6 +58,10 @@ struct SumsLeft {
   jg_conv_reduction sums = {};
   std::vector<at::Tensor> held;
 };
+// The most scratch that is held for it through the input gradient and the exchange. A launch of 4 to 10 us less is worth the workgroups'
+// partials (up to 38 MB), but not the copies of both tensors that fp32 layers on sums of bf16 parts have beside them: 3.1 GB for 1 x 64 -> 64 of
+// 2048^2, which the input gradient (1.1 GB) and its own copies (1.6) have else the place of.
+constexpr size_t kMostHeld = size_t(64) << 20;
 
 class Step {
  public:
@@ -69,7 +73,8 @@ class Step {
         elem_(elem_size), code_(code), own_(*reinterpret_cast<const jg_halo_geom*>(own)),
         theirs_(*reinterpret_cast<const jg_halo_geom*>(theirs)), same_(same), desc_(*reinterpret_cast<const jg_conv_desc*>(desc)),
         nbytes_(nbytes), recv_fwd_(strips(recv_fwd)), recv_bwd_(strips(recv_bwd)), send_fwd_(strips(send_fwd)),
-        send_bwd_(strips(send_bwd)), beside_(jg_halo_fold_border_takes_sums(&theirs_, code) == 1), fold_(try_fold) {}
+        send_bwd_(strips(send_bwd)), beside_(nbytes_[JG_CONV_WGRAD] <= kMostHeld && jg_halo_fold_border_takes_sums(&theirs_, code) == 1),
+        fold_(try_fold) {}
 
   bool sends() const { return !send_fwd_.empty(); }
 
@@ -123,7 +128,7 @@ class Step {
         if (need_x && beside_ && fold_.load(std::memory_order_relaxed)) {  // the last of the sums beside the border cells, in `finish`
           rc = jg_conv_wgrad_bias_later(&later.sums, gw_t.data_ptr(), gb_t.data_ptr(), x_aug.data_ptr(), g.data_ptr(), &desc_, code_,
                                         address(ws), nbytes_[JG_CONV_WGRAD], s);
-          later.held = {ws, gw_t, gb_t};
+          if (later.sums.kind != 0) later.held = {ws, gw_t, gb_t};
         } else {
           rc = jg_conv_wgrad_bias(gw_t.data_ptr(), gb_t.data_ptr(), x_aug.data_ptr(), g.data_ptr(), &desc_, code_, address(ws),
                                   nbytes_[JG_CONV_WGRAD], s);
@@ -157,8 +162,12 @@ class Step {
         }
       }
       if (later.sums.kind != 0) {
-        if (folded) left = py::cast(std::move(later));
-        else check(jg_conv_reduce(&later.sums, s), "jg_conv_reduce");
+        if (folded) {
+          left = py::cast(std::move(later));
+        } else {
+          check(jg_conv_reduce(&later.sums, s), "jg_conv_reduce");
+          later.held.clear();
+        }
       }
       if (!folded) {
         const at::Tensor need = at::empty(padded_, g.options());

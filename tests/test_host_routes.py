@@ -121,6 +121,39 @@ def test_the_python_route_writes_the_input_gradient_to_its_owners_for_every_type
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ci, co, size, dtype, held", [
+    (40, 72, (97, 120), torch.bfloat16, True),     # partials alone
+    (24, 40, (480, 500), torch.float32, False),    # sums of bf16 parts: copies of both tensors beside the partials
+    (8, 8, (24, 64, 96), torch.float32, False),    # all part products in one block: no sums are left
+], ids=str)
+def test_a_step_holds_no_more_of_the_weight_gradients_scratch_than_the_sums_left_need(ci, co, size, dtype, held):
+    """The weight gradient's scratch makes room for the input gradient, unless sums over it are left for the border's launch: then it is
+    64 MiB at most."""
+    dev, n, lib = torch.device("cuda:0"), len(size), _lib.load()
+    kernel, ones, ranks, mesh = (3,) * n, (1,) * n, (0,) * n, (2,) * n
+    x_shape, w_shape = (1, ci, *size), (co, ci, *kernel)
+    geom = HaloGeometry.for_conv(size, kernel, ones, ones, ones, ranks, mesh)
+    assert lib.jg_halo_fold_border_takes_sums(geom.theirs().c_geom(ci), _lib.dtype_code(dtype)) == 1
+    step = jc._step(x_shape, dtype, w_shape, ones, ones, ones, ranks, mesh, 1, True)
+    local = jc._local_padding(ones, mesh)
+    ws_x, ws_w = (jc._launch_for(op, dtype, x_shape[:2] + geom.padded, w_shape, ones, local, ones, 1).nbytes for op in (1, 2))
+    mk = lambda *shape: torch.randn(*shape, device=dev).to(dtype)  # noqa: E731
+    x_aug, w, g = mk(*x_shape[:2], *geom.padded), mk(*w_shape), mk(1, co, *size)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    parts = step.backward(g, x_aug, w, True, True, True, _lib.stream_handle(dev))
+    peak = torch.cuda.max_memory_allocated() - before
+    gx, gw, gb, send, folded, left = parts
+    assert folded and (left is not None) == held
+    step.finish(gx, folded, {}, _lib.stream_handle(dev), left)
+    results = sum(t.numel() * t.element_size() for t in (gx, gw, gb, *send.values()))
+    room = 6 << 20  # the allocator leaves up to 1 MiB behind a block of more than that as part of it
+    assert peak <= room + (ws_w + ws_x + results if held else max(ws_w + gw.numel() * 4, ws_x + results))
+    assert not held or ws_w <= 64 << 20
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_norms_and_rings_by_the_native_and_the_python_route_agree_bit_for_bit(dtype, monkeypatch):
     from jigsaw_amd import attention, groupnorm, layernorm
