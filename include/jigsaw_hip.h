@@ -596,7 +596,7 @@ int jg_conv_wgrad_bias(void* gw, void* gb, const void* x, const void* g,
  * nothing. jg_conv_reduce or jg_halo_fold_border_reduce_3d does it, on a stream ordered behind the call and with the bits of
  * jg_conv_wgrad_bias; until then workspace, gw and gb stay where they are. */
 typedef struct jg_conv_reduction {
-  int32_t kind, dtype; /* the library's own, as all of it */
+  int32_t kind, dtype; /* the library's own, as all of it: what no call has set is JG_ERR_BAD_ARG */
   const float* part;
   const float* bias_part;
   void* gw;

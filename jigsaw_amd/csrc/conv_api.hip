@@ -227,14 +227,30 @@ extern "C" int jg_conv_wgrad_bias_later(jg_conv_reduction* later, void* gw, void
   return wgrad_bias(later, gw, gb, x, go, desc, dtype, workspace, workspace_bytes, stream);
 }
 
+int jg::check_conv_reduction(const jg_conv_reduction& r, const char* who) {
+  if (r.kind == CONV_REDUCE_NONE) return JG_OK;
+  const bool tiles = r.kind == CONV_REDUCE_TILES;
+  JG_REQUIRE(tiles || r.kind == CONV_REDUCE_F32, "%s: unknown kind of sums %d", who, r.kind);
+  JG_REQUIRE(tiles ? known(r.dtype) : r.dtype == JG_F32, "%s: sums of dtype %d", who, r.dtype);
+  JG_REQUIRE(r.part != nullptr && r.gw != nullptr && (!tiles || r.gb == nullptr || r.bias_part != nullptr), "%s: sums with a NULL pointer", who);
+  const bool positive = r.runs > 0 && r.slots > 0 && r.rows > 0 && r.cols > 0 && r.ci_step > 0 && r.ci_blocks > 0 && r.cin > 0 && r.cout > 0;
+  JG_REQUIRE(positive, "%s: sums of sizes that no weight gradient leaves", who);
+  const bool blocks = tiles ? r.sub >= 0 && r.sub <= 2 && r.pairs > 0 && r.KD > 0 && (r.npairs == 1 || r.npairs == 6) && r.runs % (36ll * r.pairs) == 0 &&
+                                  (r.gb == nullptr || (r.bias_cout > 0 && r.bias_parts >= 1 && r.bias_parts <= 3))
+                            : (long long)r.rows * r.cols % CONV_F32_VALUES == 0 && r.runs % ((long long)r.rows * r.cols / CONV_F32_VALUES) == 0;
+  JG_REQUIRE(blocks, "%s: sums of sizes that no weight gradient leaves", who);
+  return JG_OK;
+}
+
 int jg::conv_reduce(const jg_conv_reduction& later, hipStream_t s) {
   if (later.kind == CONV_REDUCE_TILES) return tiles_reduce(later, s);
   if (later.kind == CONV_REDUCE_F32) return f32_reduce(later, s);
-  JG_REQUIRE(later.kind == CONV_REDUCE_NONE, "jg_conv_reduce: unknown kind %d", later.kind);
   return JG_OK;
 }
 
 extern "C" int jg_conv_reduce(const jg_conv_reduction* later, void* stream) {
   JG_REQUIRE(later != nullptr, "jg_conv_reduce: NULL pointer");
+  const int rc = jg::check_conv_reduction(*later, "jg_conv_reduce");
+  if (rc) return rc;
   return jg::conv_reduce(*later, static_cast<hipStream_t>(stream));
 }

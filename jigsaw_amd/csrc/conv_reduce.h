@@ -154,7 +154,9 @@ __device__ __forceinline__ void reduce_conv_f32(const jg_conv_reduction& p, unsi
   if (j == p.ci_step * 9 && block % p.ci_blocks == 0 && p.gb != nullptr) static_cast<float*>(p.gb)[co] = sum;
 }
 
-// Does what `later` holds, by itself.
+// Whether `later` is something that the weight gradient can have left: an error where it is not (conv_api.hip).
+int check_conv_reduction(const jg_conv_reduction& later, const char* who);
+// Does what `later`, so checked, holds, by itself.
 int conv_reduce(const jg_conv_reduction& later, hipStream_t s);
 
 }  // namespace jg

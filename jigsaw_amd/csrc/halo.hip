@@ -1683,6 +1683,8 @@ extern "C" int jg_halo_fold_border_3d(void* gx, const void* const strips[27],
 extern "C" int jg_halo_fold_border_reduce_3d(void* gx, const void* const strips[27], const jg_halo_geom* geom, int dtype,
                                              const jg_conv_reduction* later, void* stream) {
   JG_REQUIRE(later != nullptr, "jg_halo_fold_border_reduce_3d: NULL pointer");
+  const int rc = jg::check_conv_reduction(*later, "jg_halo_fold_border_reduce_3d");
+  if (rc) return rc;
   return fold_border(gx, strips, geom, dtype, later, stream);
 }
 

@@ -88,6 +88,35 @@ def test_misaligned_chunks_are_refused_without_a_gpu(which, d):
         assert rc == -2 and b"aligned" in lib.jg_last_error()
 
 
+class _ConvReduction(ctypes.Structure):
+    _fields_ = ([(n, ctypes.c_int32) for n in ("kind", "dtype")] + [(n, ctypes.c_void_p) for n in ("part", "bias_part", "gw", "gb")]
+                + [(n, ctypes.c_int32) for n in ("runs", "sub", "slots", "npairs", "pairs", "rows", "cols", "ci_step", "ci_blocks", "KD",
+                                                 "cin", "cout", "bias_cout", "bias_parts")])
+
+
+@pytest.mark.parametrize("wrong", [
+    {"kind": 3}, {"kind": -1}, {"dtype": 7}, {"kind": 2}, {"part": None}, {"gw": None}, {"bias_part": None}, {"runs": 0}, {"runs": 35}, {"sub": 3},
+    {"slots": 0}, {"npairs": 2}, {"pairs": 0}, {"rows": 0}, {"cols": -1}, {"ci_step": 0}, {"ci_blocks": 0}, {"KD": 0}, {"cin": 0}, {"cout": 0},
+    {"bias_cout": 0}, {"bias_parts": 4}, {"kind": 2, "dtype": 0, "rows": 1, "cols": 1},
+], ids=str)
+def test_sums_that_no_weight_gradient_left_are_refused_without_a_gpu(wrong):
+    """jg_conv_reduce and jg_halo_fold_border_reduce_3d take a descriptor that the weight gradient has filled, and none else."""
+    lib, at = jigsaw_amd.load(), 0x1000
+    good = dict(kind=1, dtype=1, part=at, bias_part=at, gw=at, gb=at, runs=36, sub=2, slots=4, npairs=1, pairs=1, rows=32, cols=1, ci_step=32,
+                ci_blocks=1, KD=1, cin=8, cout=8, bias_cout=8, bias_parts=1)
+    geom = _lib.HaloGeom()
+    geom.planes = 8
+    for a, (size, halo) in enumerate(((1, 0), (8, 1), (8, 1))):
+        geom.size[a], geom.lo[a], geom.hi[a] = size, halo, halo
+    left = _ConvReduction(**{**good, **wrong})
+    strips = _lib.VoidP27()
+    assert lib.jg_conv_reduce(ctypes.byref(left), None) == -1 and b"jg_conv_reduce" in lib.jg_last_error()
+    rc = lib.jg_halo_fold_border_reduce_3d(ctypes.c_void_p(at), strips, geom, left.dtype if wrong.get("dtype") != 7 else 1, ctypes.byref(left), None)
+    assert rc == -1 and b"sums" in lib.jg_last_error()
+    none = _ConvReduction()
+    assert lib.jg_conv_reduce(ctypes.byref(none), None) == 0  # nothing left
+
+
 def test_weight_gradient_of_large_operands_keeps_its_kernel_without_a_gpu():
     """jg_proj_tn on bf16 operands of 2^32 bytes and more: the matrix-core kernel, which asks for its workspace (the
     one-product-at-a-time kernel needs none)."""
