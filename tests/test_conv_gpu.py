@@ -945,16 +945,31 @@ def test_fp32_layers_of_few_channels_are_as_exact_as_their_kernels_in_every_dire
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("n, c_in, c_out, size, mesh", [
-    (2, 32, 32, (40, 72), (2, 2)),      # 36 runs of sums in pieces of four, beside the border
-    (1, 5, 7, (9, 11), (3, 3)),         # a single workgroup's partials, odd rows
-    (2, 64, 64, (40, 70), (2, 2)),      # 144 runs
-    (1, 96, 80, (24, 66), (3, 1)),      # several blocks of channels, no neighbour across W
-    (1, 24, 7, (6, 20, 18), (2, 2, 2)),  # three depth taps
-    (4, 40, 8, (300, 310), (3, 3)),     # a border of more blocks than the chip holds: launches of their own
+@pytest.mark.parametrize("n, c_in, c_out, size, mesh, beside", [
+    (2, 32, 32, (40, 72), (2, 2), True),      # 36 runs of sums in pieces of four, beside the border
+    (1, 5, 7, (9, 11), (3, 3), True),         # a single workgroup's partials, odd rows
+    (2, 64, 64, (40, 70), (2, 2), True),      # 144 runs
+    (1, 96, 80, (24, 66), (3, 1), True),      # several blocks of channels, no neighbour across W
+    (1, 24, 7, (6, 20, 18), (2, 2, 2), True),  # three depth taps
+    (4, 40, 8, (300, 310), (3, 3), True),     # long rows and columns; an odd number of whole octets of channels
+    (4, 96, 8, (700, 24), (3, 3), False),     # a border of more blocks than the chip holds (8 a compute unit): launches of their own
 ])
-def test_sums_left_for_the_border_launch_have_the_bits_of_their_own(n, c_in, c_out, size, mesh, dtype, dev):
+def test_sums_left_for_the_border_launch_have_the_bits_of_their_own(n, c_in, c_out, size, mesh, beside, dtype, dev, monkeypatch):
     """Weight and bias gradient of the halo convolution, whose last sums run beside the border cells, == conv_nd_weight's."""
+    ways, step_for = [], jc._step_for
+
+    class Watched:  # a native step that says whether it left sums
+        def __init__(self, step):
+            self.step = step
+
+        def __getattr__(self, name):
+            return getattr(self.step, name)
+
+        def finish(self, *a):
+            ways.append(a[-1] is not None)
+            return self.step.finish(*a)
+
+    monkeypatch.setattr(jc, "_step_for", lambda *a: Watched(step_for(*a)))
     ns, gen = len(size), torch.Generator().manual_seed(5)
     k, ones = (3,) * ns, (1,) * ns
     rank = tuple(1 if m == 3 else 0 for m in mesh)
@@ -978,6 +993,12 @@ def test_sums_left_for_the_border_launch_have_the_bits_of_their_own(n, c_in, c_o
     from jigsaw_amd.halo import halo_fold
 
     assert torch.equal(gx, halo_fold(need, recv_b, geom))
+    assert ways == [beside]
+    assert _lib.load().jg_halo_fold_border_takes_sums(geom.theirs().c_geom(n * c_in), _lib.dtype_code(dtype)) == beside
+    # y, rounded once: 2^-9 and 2^-12 of a value at most; fp32 sums of at most 864 products are off by 1e-6 at the most
+    conv = torch.nn.functional.conv2d if ns == 2 else torch.nn.functional.conv3d
+    exact = conv(x_aug.detach().cpu().double(), w.cpu().double(), b.cpu().double(), padding=lp)
+    assert rel_l2(y, exact) < {torch.bfloat16: 2**-9, torch.float16: 2**-12, torch.float32: 0.0}[dtype] + 1e-6
 
 
 @pytest.mark.gpu

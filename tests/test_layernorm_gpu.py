@@ -167,6 +167,35 @@ def test_layernorm_rows_that_end_in_half_an_octet(cols, dtype, dev):
     assert (guard[x.numel():] == 7).all()
 
 
+@pytest.mark.parametrize("cols,dtype", [(12, torch.bfloat16), (76, torch.float16), (132, torch.bfloat16), (164, torch.bfloat16)],
+                         ids=lambda v: str(v).replace("torch.", ""))
+def test_layernorm_writes_fp32_from_16_bit_rows_that_end_in_half_an_octet(cols, dtype, dev):
+    """As under autocast, from 2^22 elements on: x, whose rows start at multiples of 8 bytes, in another type than what is written; 164 columns
+    are past the widest fp32 row that the kernel for these rows writes."""
+    rows = (1 << 22) // cols + 3
+    gen = torch.Generator().manual_seed(cols)
+    x = (torch.randn(rows, cols, generator=gen) * 3 + 1.5).to(dtype)
+    w, b = 1 + 0.2 * torch.randn(cols, generator=gen), 0.2 * torch.randn(cols, generator=gen)
+    g = torch.randn(rows, cols, generator=gen)
+    xd, wd, bd = x.double(), w.double(), b.double()
+    # one shard of two whose other half holds the same values: its statistics are those of these columns
+    mean, var = xd.mean(-1, keepdim=True), xd.var(-1, unbiased=False, keepdim=True)
+    gxn = g.double() * wd
+    x_hat = (xd - mean) / (var + 1e-5).sqrt()
+    grp = ShardGroup(2, [[mean], [var], [gxn.mean(-1, keepdim=True)], [(gxn * x_hat).sum(-1, keepdim=True)]])
+    xr, wr, br = (t.to(dev).requires_grad_() for t in (x, w, b))
+    with torch.autocast("cuda", dtype=dtype):
+        y = jl.layer_norm(xr, wr, br, grp, 1e-5)
+    assert y.dtype == torch.float32 and grp.calls == ["avg", "avg"]
+    y.backward(g.to(dev))
+    assert xr.grad.dtype == dtype and wr.grad.dtype == br.grad.dtype == torch.float32
+    gx = (gxn - gxn.mean(-1, keepdim=True) - x_hat * (gxn * x_hat).mean(-1, keepdim=True)) / (var + 1e-5).sqrt()
+    # fp32 throughout: chains of some 10 roundings along a row and some 40 down the columns, 6e-8 each; x's gradient is rounded to its type
+    once = 2**-9 if dtype == torch.bfloat16 else 2**-12
+    for got, want, off in ((y, x_hat * wd + bd, 0.0), (xr.grad, gx, once), (wr.grad, (g.double() * x_hat).sum(0), 0.0), (br.grad, g.double().sum(0), 0.0)):
+        assert rel_l2(got, want) < off + 1e-5
+
+
 def test_layernorm_under_autocast_returns_fp32_and_leaf_dtype_grad(dev):
     """LayerNorm under autocast computes in fp32 (reference: tests/test_autocast.py:265-292)."""
     torch.manual_seed(2)
