@@ -17,7 +17,8 @@
 // the 0.16 PFLOP/s of this instruction, but the parts are written and read, in launches of their own, and a step there is 16 channels of
 // six products whatever the layer has. Batch 4, 3 -> 16 channels, 256^2 (that : this): forward 28 : 9.5 us, gradients of the
 // weight and bias 46 : 10.5 and their sums beside the border cells, input gradient 55 : 13, 14 launches : 6. What bounds it there: latency, at one or two stages a workgroup;
-// with many channels the instruction's rate, 74 of 157 TFLOP/s at 20 -> 20 channels, 8 x 500^2. f32_conv_supported has the line
+// with many channels the instruction's rate: forward, 105 of 157 TFLOP/s at 8 x 64 -> 64, 512^2 (58 at 8 x 20 -> 20, 500^2, where 12 of a
+// block's 32 produced channels do not exist). f32_conv_supported has the line
 // between the two. Against float64 no result is further off than the three parts' (relative, 16 channels: y 1.9e-7 : 2.5e-7).
 #include "conv_common.h"
 #include "conv_reduce.h"
@@ -481,23 +482,26 @@ bool f32_conv_supported(const ConvGeom& g, int dtype) {
     if (g.s[a] != 1 || g.d[a] != 1 || g.p[a] > g.k[a] - 1 || g.out[a] < 1) return false;
   const long long tiles = g.batch * ((std::max(g.in[1], g.out[1]) + GR - 1) / GR) * ((std::max(g.in[2], g.out[2]) + TW - 1) / TW);
   if (tiles >= (1ll << 22) || (g.cin + 13) / 14 * ((g.cout + 15) / 16) >= 65536) return false;
-  // Against sums of bf16 parts, forward + both gradients, us (this : that). Up to 16 channels on one side:
-  //   4 x 3 -> 16, 256^2 60 : 134   8 x 16 -> 16, 512^2 640 : 708   2 x 12 -> 100, 150^2 154 : 252   8 x 3 -> 64, 512^2 920 : 1829
+  // Against sums of bf16 parts: the traced kernels of forward, weight and bias gradient and input gradient at padding 1, us (this : that).
+  // Up to 16 channels on one side:
+  //   4 x 3 -> 16, 256^2 36 : 122     8 x 16 -> 16, 512^2 547 : 780   2 x 12 -> 100, 150^2 120 : 219  8 x 3 -> 64, 512^2 534 : 1687
+  //   8 x 16 -> 128, 256^2 918 : 956  8 x 128 -> 16, 256^2 772 : 972  but 4 x 15 -> 18, 512^2 418 : 396
   // and a layer whose workgroups are fewer than the compute units is bound by its launches, 6 here and 12 there, and by stages of which
   // a compute unit has one at a time. With 65 to 128 channels on one side (more have not been
-  // measured) and up to 64 on the other that holds up to three workgroups for four compute units (kernels alone, without the launches' gaps):
-  //   2 x 24 -> 24, 200^2 108 : 153   1 x 64 -> 64, 100^2 161 : 225   1 x 64 -> 64, 180^2 204 : 250   2 x 48 -> 48, 150^2 193 : 227
-  //   1 x 17 -> 65, 40^2 98 : 130     8 x 17 -> 80, 64^2 137 : 155    2 x 20 -> 70, 128^2 131 : 155   1 x 40 -> 80, 256 x 128 170 : 196
-  //   2 x 127 -> 40, 48^2 175 : 215   2 x 48 -> 100, 64^2 161 : 189   4 x 40 -> 66, 48 x 90 144 : 192  1 x 64 -> 80, 128^2 172 : 180
-  //   1 x 32 -> 128, 128^2 180 : 181  but 1 x 128 -> 17, 128 x 256 (256 workgroups) 206 : 196, 3 x 80 -> 128, 64^2 236 : 226
-  // Beyond, their rate wins:
-  //   4 x 32 -> 32, 256^2 298 : 231   2 x 64 -> 64, 180^2 312 : 228   1 x 96 -> 96, 128^2 229 : 220   8 x 64 -> 64, 512^2 6060 : 3851
-  //   4 x 17 -> 64, 256^2 367 : 313   8 x 20 -> 20, 500^2 1123 : 1074  but 4 x 20 -> 20, 300^2 248 : 259   8 x 28 -> 31, 300^2 553 : 593
-  // Within the line the parts are faster in one direction or other of large layers: where 9 to 16 channels go into more than 32
-  // (16 fill the parts' step; this has two stages of 8 and half of its rate), and in the weight gradient of 15 to 21 input channels, which need a
-  // second block of columns here (forward, weight gradient, input gradient; all but the last with staging since made 5 to 20 % faster here):
-  //   8 x 16 -> 128, 256^2 242 : 168, 524 : 509, 342 : 418   8 x 128 -> 16, 256^2 301 : 365, 409 : 491, 305 : 224
-  //   4 x 15 -> 18, 512^2 124 : 111, 287 : 151, 117 : 163    8 x 16 -> 16, 256^2 41 : 66, 77 : 88, 49 : 76
+  // measured) and up to 64 on the other that holds up to three workgroups for four compute units:
+  //   2 x 24 -> 24, 200^2 100 : 137   1 x 64 -> 64, 100^2 132 : 159   1 x 64 -> 64, 180^2 168 : 183   2 x 48 -> 48, 150^2 158 : 174
+  //   1 x 17 -> 65, 40^2 87 : 125     8 x 17 -> 80, 64^2 121 : 156    2 x 20 -> 70, 128^2 116 : 162   1 x 40 -> 80, 256 x 128 152 : 206
+  //   2 x 127 -> 40, 48^2 160 : 201   2 x 48 -> 100, 64^2 147 : 192   4 x 40 -> 66, 48 x 90 130 : 195 1 x 64 -> 80, 128^2 157 : 184
+  //   1 x 32 -> 128, 128^2 165 : 183
+  // Beyond, their rate wins the more the larger the layer is; next to the line the two are within 14 % of each other:
+  //   8 x 64 -> 64, 512^2 5308 : 3687 2 x 64 -> 64, 180^2 280 : 216   8 x 20 -> 20, 500^2 986 : 895   4 x 32 -> 32, 256^2 222 : 213
+  //   4 x 20 -> 20, 300^2 218 : 222   8 x 28 -> 31, 300^2 455 : 477   4 x 17 -> 64, 256^2 279 : 299   1 x 96 -> 96, 128^2 207 : 223
+  //   3 x 80 -> 128, 64^2 220 : 233   1 x 128 -> 17, 128 x 256 (256 workgroups) 175 : 198
+  // Within the line the parts are faster in one direction or other: where 16 channels go into many more (they fill the parts' step; this
+  // has two stages of 8), and in weight gradients that need a second block of columns here, 15 input channels and more (y, gw, gx):
+  //   8 x 16 -> 128, 256^2 209 : 143, 485 : 482, 224 : 331            8 x 128 -> 16, 256^2 219 : 335, 352 : 497, 201 : 140
+  //   4 x 15 -> 18, 512^2 99 : 102, 242 : 151, 78 : 143               2 x 48 -> 48, 150^2 42 : 58, 75 : 58, 41 : 58
+  //   but 8 x 16 -> 16, 256^2 39 : 61, 74 : 87, 37 : 62               8 x 17 -> 80, 64^2 20 : 32, 42 : 45, 59 : 79
   // Those directions stay here too: the parts are less exact in all of them. Relative error against float64, 16 -> 128: y 1.6e-7 :
   // 2.5e-7, gw 6.4e-8 : 2.0e-7, input gradient of 128 from 16 1.6e-7 : 2.5e-7 (3 channels 0.94e-7 : 1.13e-7).
   const int few = std::min(g.cin, g.cout), many = std::max(g.cin, g.cout);
