@@ -29,8 +29,8 @@ __device__ __forceinline__ void store_gradient(void* out, size_t at, float v) {
 // lie behind each other), and gb the same over the bias partials. A workgroup owns a run of 256 >> sub values of a
 // block's partial (a tap, a pair, four registers and 64 >> sub lanes of the kernel that wrote it), a lane four of them; 8
 // wavefronts take 8 << sub partials at a time in chains of their own and the sums are added in a fixed order
-// (deterministic). What bounds it is the latency of the chains, 16-byte loads, eight in flight a lane: a block of 32 x 32 is 36 runs of 256 values, which left most of the chip idle: 6 x 26 -> 27 of
-// 197 x 140 12.4 us, cut in four 6.6.
+// (deterministic). What bounds it is the latency of the chains, 16-byte loads, eight in flight a lane. A block of 32 x 32 is 36 runs
+// of 256 values, which left most of the chip idle: 6 x 26 -> 27 of 197 x 140 took 12.4 us, and takes 6.6 cut in four.
 // The workgroups behind those of the last block add up bias partials, 16 channels each, four partials a wavefront at a time.
 template <int DT>
 __device__ __forceinline__ void reduce_conv_tiles(const jg_conv_reduction& p, unsigned block, ConvReduceShared& shared) {

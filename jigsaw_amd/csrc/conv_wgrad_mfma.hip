@@ -936,8 +936,8 @@ Plan plan_of(const ConvGeom& g, int parts) {
   if (n >= 8) n = n / 8 * 8;
   if (n > stages) n = stages;
   if (n < 1) n = 1;
-  // No more than the walks need: 1080 stages in walks of four are 270 workgroups, of 336 that the rule asks for 66 wrote
-  // a partial of nothing.
+  // No more than the walks need, but for up to seven that make the number a multiple of the XCDs: 1080 stages in walks of four are 270
+  // workgroups and 272 are launched, of the 336 that the rule asks for 66 wrote a partial of nothing.
   const long long walk = (stages + n - 1) / n, busy = (stages + walk - 1) / walk;
   if (n >= 8) n = std::min(n, (busy + 7) / 8 * 8);
   else n = busy;

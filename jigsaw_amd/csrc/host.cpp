@@ -59,8 +59,8 @@ struct SumsLeft {
   std::vector<at::Tensor> held;
 };
 // The most scratch that is held for it through the input gradient and the exchange. A launch of 4 to 10 us less is worth the workgroups'
-// partials (up to 38 MB), but not the copies of both tensors that fp32 layers on sums of bf16 parts have beside them: 3.1 GB for 1 x 64 -> 64 of
-// 2048^2, which the input gradient (1.1 GB) and its own copies (1.6) have else the place of.
+// partials (up to 38 MB below 1000 channels), but not the copies of both tensors that fp32 layers on sums of bf16 parts have beside
+// them: 3.1 GB for 1 x 64 -> 64 of 2048^2, which the input gradient (1.1 GB) and its own copies (1.6) have else the place of.
 constexpr size_t kMostHeld = size_t(64) << 20;
 
 class Step {

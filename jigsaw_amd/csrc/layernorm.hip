@@ -649,6 +649,7 @@ __global__ __launch_bounds__(kThreads, CH == 1 ? 4 : 1) void ln_plain_bwd_kernel
 // partial_bwd / bwd_apply, us:
 //   262144 x 132 bf16 73 -> 30 / 88 -> 63 / 82 -> 43 / 65 -> 38   30000 x 1540 bf16 39 -> 25 / 61 -> 57 / 122 -> 49 / 55 -> 48
 //   200000 x 76 fp32 52 -> 16 / 54 -> 32 / 48 -> 23 / 42 -> 31    51966 x 652 fp32 41 -> 33 / 80 / 75 -> 68 / 66
+
 // 8 columns as they lie in memory (16 or 32 bytes), converted later: a kernel can then request the rows of its
 // next round before it turns to the arithmetic of the current one, and the loads stay in the air meanwhile.
 template <int DT, bool HALF>
@@ -1028,11 +1029,12 @@ bool rows_ok(long long rows, long long cols, int dtype) {
   const long long least = 1ll << (dtype == JG_F32 ? 22 : 20);
   return cols > kPlainVec && cols % kPlainVec == 4 && plain_chunks(cols) <= kPlainChunks && rows >= least / cols;
 }
-// The two kernels that write rows, where the walking kernel is the better one (it : rows in registers, apply / bwd_apply, us): fp32 rows that
-// give most lanes of a walking wavefront their 16 bytes, which cover whole lines behind each other while an octet a lane touches each line twice:
+// The two kernels that write rows keep the walking kernel where it is the better one (it : rows in registers, apply / bwd_apply, us): fp32 rows
+// that give most lanes of a walking wavefront their 16 bytes, which cover whole lines behind each other while an octet a lane touches each line
+// twice. One line for both directions, between 132 and 180 columns; the forward of the widest rows loses 6 % by it.
 //   100000 x 132 31 : 29 / 28 : 27   100000 x 180 35 : 38 / 34 : 35   100000 x 252 55 : 61 / 47 : 58   100000 x 388 87 : 100 / 72 : 93
-//   60000 x 516 75 : 75 / 63 : 70    40000 x 1300 126 : 119 / 108 : 113   4000 x 1028 10.3 : 13.8 / 10.0 : 11.2
-// and the forward's 16-bit rows whose second chunk is less than half full:
+//   60000 x 516 75 : 75 / 63 : 70    40000 x 1300 126 : 119 / 108 : 113
+// And the forward's 16-bit rows whose second chunk is less than half full:
 //   60000 x 516 49 : 52   51966 x 652 46 : 49   60000 x 772 66 : 60   100000 x 508 76 : 66
 bool rows_written_ok(long long rows, long long cols, int out_dtype, bool forward) {
   if (!rows_ok(rows, cols, out_dtype)) return false;
@@ -1130,9 +1132,10 @@ extern "C" int jg_ln_partial_fwd2(float* mean, float* mean2, float* var, const v
   const int G = in_regs ? plain_group(cols) : 0, blocks = in_regs ? plain_blocks(rows, cols, 8192) : 0;
 #define JG_GO(DT)                                                                                  \
   if (in_regs)                                                                                     \
-    with_sharded_row_shape<4>(cols, [&](auto ch, auto u, auto half) {                                                 \
-      ln_partial_fwd_rows_kernel<DT, decltype(ch)::value, decltype(u)::value, decltype(half)::value>                      \
-          <<<blocks, kThreads, 0, s>>>(mean, mean2, var, static_cast<const Elem<DT>::T*>(x), rows, (int)cols, G); \
+    with_sharded_row_shape<4>(cols, [&](auto ch, auto u, auto half) {                              \
+      ln_partial_fwd_rows_kernel<DT, decltype(ch)::value, decltype(u)::value, decltype(half)::value> \
+          <<<blocks, kThreads, 0, s>>>(mean, mean2, var, static_cast<const Elem<DT>::T*>(x), rows, \
+                                       (int)cols, G);                                              \
     });                                                                                            \
   else                                                                                             \
     ln_partial_fwd_kernel<DT><<<row_grid(rows), kThreads, 0, s>>>(                                 \
@@ -1370,13 +1373,16 @@ extern "C" int jg_ln_bwd_apply(void* gx, const void* g, const void* x_hat, const
     const bool v = vec_aligned(g, cols, DT) && vec_aligned(x_hat, cols, DT) &&             \
                    vec_aligned(gx, cols, DT);                                              \
     const bool vw = vec_aligned(w, cols, DT);                                              \
-    if (rows_written_ok(rows, cols, DT, false) && aligned16(gx) && aligned16(g) && aligned16(x_hat) && aligned16(w)) { \
-      const int G = plain_group(cols), blocks = plain_blocks(rows, cols, 2048);                  \
-      with_sharded_row_shape<2>(cols, [&](auto ch, auto u, auto half) {                                       \
-        ln_bwd_apply_rows_kernel<DT, decltype(ch)::value, decltype(u)::value, decltype(half)::value>              \
+    if (rows_written_ok(rows, cols, DT, false) && aligned16(gx) && aligned16(g) &&         \
+        aligned16(x_hat) && aligned16(w)) {                                                \
+      const int G = plain_group(cols), blocks = plain_blocks(rows, cols, 2048);            \
+      with_sharded_row_shape<2>(cols, [&](auto ch, auto u, auto half) {                    \
+        ln_bwd_apply_rows_kernel<DT, decltype(ch)::value, decltype(u)::value,              \
+                                 decltype(half)::value>                                    \
             <<<blocks, kThreads, 0, s>>>(static_cast<T*>(gx), static_cast<const T*>(g),    \
                                          static_cast<const T*>(x_hat), static_cast<const T*>(w), \
-                                         mean_gxn, dot_gxn_xhat, std, rows, (int)cols, inv_n, G); \
+                                         mean_gxn, dot_gxn_xhat, std, rows, (int)cols,     \
+                                         inv_n, G);                                        \
       });                                                                                  \
     } else                                                                                 \
     ln_bwd_apply_kernel<DT><<<row_grid(rows), kThreads, 0, s>>>(                           \
