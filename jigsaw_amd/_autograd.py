@@ -6,6 +6,12 @@ import torch
 from torch import _functorch
 
 
+def native_nodes() -> bool:
+    """Whether a layer may leave its autograd node to the native host module: not under a functorch transform, in a trace or in
+    a compiled graph, which know the Python functions."""
+    return not (torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling())
+
+
 class PositionalFunction(torch.autograd.Function):
     """A ``torch.autograd.Function`` with ``setup_context`` whose ``apply`` takes positional arguments as they are.
 

@@ -18,6 +18,7 @@ that talks to other ranks), and assembles the padded tile in one pass.
 
 from __future__ import annotations
 
+import copy
 import ctypes
 import itertools
 import math
@@ -28,7 +29,7 @@ from typing import Any, Protocol
 import torch
 
 from . import _lib
-from ._autograd import PositionalFunction
+from ._autograd import PositionalFunction, native_nodes
 from .halo import (HaloGeometry, halo_assemble, halo_fold, halo_fold_border_, halo_gather_axis, halo_pack,
                    halo_scatter_add_axis, new_strips, spans_fit_the_strips, strip_table)
 
@@ -1291,9 +1292,62 @@ def _cast_to_autocast_dtype(*tensors):
     return tuple(t if t is None or not t.is_floating_point() else t.to(dt) for t in tensors)
 
 
+class _Received:
+    """The exchange of a layer whose forward strips have travelled already."""
+
+    def __init__(self, exchange, recv: dict) -> None:
+        self._exchange, self._recv = exchange, recv
+
+    def forward(self, send: dict) -> dict:
+        return self._recv
+
+    def __getattr__(self, name):
+        return getattr(self._exchange, name)
+
+
+def _backward_without_plan(g, x_aug, weight, need_x, need_w, need_b, local_in_spatial, stride, padding, dilation, spatial_groups, channel_group, config):
+    """The backward of a layer whose native node declined what it got (saved tensors that came back in another layout)."""
+    if x_aug.dtype != weight.dtype:
+        x_aug = x_aug.to(weight.dtype)
+    return conv_halo_nway_backward(g, x_aug, weight, stride, padding, dilation, local_in_spatial, spatial_groups, channel_group, config,
+                                   need=(need_x, need_w, need_b))
+
+
+def _fold_without_plan(part, folded, recv, weight, local_in_spatial, stride, padding, dilation, spatial_groups, channel_group, config):
+    """The last step of the backward where the neighbours' strips are not what the plan takes."""
+    ranks, sizes = _mesh_position(spatial_groups)
+    geom = HaloGeometry.for_conv(local_in_spatial, weight.shape[-config.n_spatial:], stride, padding, dilation, ranks, sizes)
+    return halo_fold_border_(part, recv, geom) if folded else halo_fold(part, recv, geom)
+
+
 class _ConvNd(PositionalFunction):
     """Autograd function of the distributed convolution
-    (jigsaw/modules/convolution/_conv/functional.py:28-169), HIP kernels inside."""
+    (jigsaw/modules/convolution/_conv/functional.py:28-169), HIP kernels inside. Layers that the native plan runs as they
+    are get a node of the native host module instead (``host.conv_apply``): the same launches, less of the host."""
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        if cls is not _ConvNd or kwargs or len(args) != 9 or not native_nodes() or torch.is_autocast_enabled():
+            return super().apply(*args, **kwargs)
+        x, w, b, stride, padding, dilation, spatial_groups, channel_group, config = args
+        if (not isinstance(padding, tuple) or (channel_group is not None and channel_group.size() != 1)
+                or config.dist_conv_fn is not conv_halo_nway or config.dist_conv_backward_fn is not conv_halo_nway_backward
+                or not getattr(config, "fused_bias_grad", False)):
+            return super().apply(*args)
+        step = _step_for(config, x.shape, x, w, stride, padding, dilation, *_mesh_position(spatial_groups))
+        host = _lib.host()
+        if step is None or type(step) is not host.Step or not host.conv_takes(step, x, w, b):
+            return super().apply(*args)
+        stream = _lib.stream_handle(x.device)
+        exchange = config.halo_exchange
+        with torch.no_grad():
+            recv = exchange.forward(step.pack(x, stream)) if step.sends else {}
+        done = host.conv_apply(step, x, recv, w, b, args[3:], stream)
+        if done is None:  # strips in another layout
+            config = copy.copy(config)
+            config.halo_exchange = _Received(exchange, recv)
+            return super().apply(*args[:8], config)
+        return done
 
     @staticmethod
     def forward(x, weight, bias, stride, padding, dilation, spatial_groups, channel_group, config):  # noqa: D102

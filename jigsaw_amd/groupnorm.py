@@ -19,6 +19,7 @@ import torch
 import torch.distributed as dist
 
 from . import _lib
+from ._autograd import native_nodes
 
 
 def _all_reduce_sum(t: torch.Tensor, groups: Sequence[Any]) -> None:
@@ -269,6 +270,11 @@ def group_norm(x, num_groups, weight=None, bias=None, spatial_groups=(), eps=1e-
     if x.numel() == 0:
         return _GroupNorm.apply(x, num_groups, weight, bias, spatial_groups, eps)[0]
     split = tuple(g for g in spatial_groups or () if g is not None and int(g.size()) > 1)
+    host = None if split or _compute_dtype(x) != x.dtype else _lib.host()
+    if host is not None and native_nodes():  # _GroupNormOutput without its Python
+        y = host.gn_apply(x, num_groups, weight, bias, float(eps), _lib.stream_handle(x.device))
+        if y is not None:
+            return y
     return _GroupNormOutput.apply(x, num_groups, weight, bias, split, eps, torch.is_grad_enabled())
 
 

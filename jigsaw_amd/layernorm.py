@@ -16,7 +16,7 @@ import torch
 import torch.distributed as dist
 
 from . import _lib
-from ._autograd import PositionalFunction
+from ._autograd import PositionalFunction, native_nodes
 
 
 def _group_size(group: Any) -> int:
@@ -189,6 +189,16 @@ class _LayerNorm(PositionalFunction):
 def layer_norm(x, weight, bias, channel_group=None, eps: float = 1e-5) -> torch.Tensor:
     """``DistributedLayerNorm.forward``'s call: ``_LayerNorm.apply(...)[0]``
     (jigsaw/modules/normalization/_layer_norm.py:363-368)."""
+    host = _lib.host() if x.is_cuda else None
+    if host is not None and native_nodes() and host.ln_takes(x, weight, bias, _compute_dtype(x)):  # _LayerNorm without its Python
+        ranks, handle = _group_size(channel_group), _lib.stream_handle(x.device)
+        mean, var, local_mean, std = host.ln_partial(x, ranks > 1, handle)
+        if ranks > 1:
+            with torch.no_grad():
+                _all_reduce(mean, "avg", channel_group)
+                host.ln_recentre(var, local_mean, mean, handle)
+                _all_reduce(var, "avg", channel_group)
+        return host.ln_output(x, mean, var, std, weight, bias, float(eps), _all_reduce, channel_group, ranks, handle)
     return _LayerNorm.apply(x, weight, bias, channel_group, eps)[0]
 
 
