@@ -448,6 +448,7 @@ constexpr unsigned long long kEmpty = ~0ull;
 //   (for 20 ms) 1158 / 2508 : 2627 / 3956
 //   2 x 64 x 512^2, 2 groups      0   40 / 49 : 39 / 52      150   89 / 315 : 91 / 342       200   355 / 533 : 293 / 463
 constexpr unsigned kPolls = 128, kPollsStarved = 48;
+constexpr long long kStreamed = 1ll << 27;  // bytes of a tensor that goes past the last-level cache
 constexpr int kMaxPartials = 2 * kThreads;  // partials of a unit: every block of the unit adds them up again
 
 struct ResidentArgs {
@@ -486,27 +487,30 @@ __device__ __forceinline__ float2 pair_of(unsigned long long v) {
   return make_float2(__uint_as_float((unsigned)v), __uint_as_float((unsigned)(v >> 32)));
 }
 
-// Sum of a per-thread value over the block, in every thread; fixed order
-template <typename T>
+// Sum of a per-thread value over kThreads threads, in every one of them; fixed order. PARTS: how many such parts the block has
+template <typename T, int PARTS = 1>
 __device__ __forceinline__ T block_total(T v) {
-  __shared__ T red[kThreads / 64];
+  __shared__ T all[PARTS * kThreads / 64];
+  T* const red = all + (PARTS > 1 ? threadIdx.x / kThreads * (kThreads / 64) : 0);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  if ((threadIdx.x & 63) == 0) all[threadIdx.x >> 6] = v;
   __syncthreads();
   return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
+template <int PARTS = 1>
 __device__ __forceinline__ float2 block_total2(float a, float b) {
-  __shared__ float2 red[kThreads / 64];
+  __shared__ float2 all[PARTS * kThreads / 64];
+  float2* const red = all + (PARTS > 1 ? threadIdx.x / kThreads * (kThreads / 64) : 0);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     a += __shfl_xor(a, o, 64);
     b += __shfl_xor(b, o, 64);
   }
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_float2(a, b);
+  if ((threadIdx.x & 63) == 0) all[threadIdx.x >> 6] = make_float2(a, b);
   __syncthreads();
   return make_float2((red[0].x + red[1].x) + (red[2].x + red[3].x), (red[0].y + red[1].y) + (red[2].y + red[3].y));
 }
@@ -620,15 +624,58 @@ __device__ __forceinline__ bool held_statistics(const ResidentArgs& q, const App
   return true;
 }
 
+// The same from the partials of a unit in LDS (at most kWhole), with the roundings of held_statistics: its tree over the lanes is (0 + 2) + (1 + 3)
+constexpr int kWhole = 4;
+template <int DT, bool BWD>
+__device__ __forceinline__ void whole_statistics(const ResidentArgs& q, const ApplyArgs& p, unsigned u, const float2 v[kWhole], float& m, float& rs,
+                                                 float& q1, float& q2) {
+  typedef typename Elem<DT>::T T;
+  q1 = q2 = 0.0f;
+  if (BWD) {
+    const int cpg = p.C / p.G;
+    float a[kWhole], b[kWhole];
+#pragma unroll
+    for (unsigned j = 0; j < kWhole; ++j) {
+      const bool there = j < q.partials;
+      const float w = there && p.weight != nullptr ? Elem<DT>::up(static_cast<const T*>(p.weight)[(u % p.G) * cpg + j / q.chunks]) : 1.0f;
+      a[j] = there ? __builtin_fmaf(w, v[j].x, 0.0f) : 0.0f;
+      b[j] = there ? __builtin_fmaf(w, v[j].y, 0.0f) : 0.0f;
+    }
+    const float inv = 1.0f / p.count;
+    rs = q.rstd[u];
+    q1 = ((a[0] + a[2]) + (a[1] + a[3])) * inv;
+    q2 = ((b[0] + b[2]) + (b[1] + b[3])) * inv;
+  } else {
+    double n[kWhole], sum[kWhole], dev[kWhole];
+#pragma unroll
+    for (unsigned j = 0; j < kWhole; ++j) {
+      const long long from = (j % q.chunks) * q.chunk_len;
+      n[j] = j >= q.partials || from >= q.S ? 0.0 : (double)(from + q.chunk_len < q.S ? q.chunk_len : q.S - from);
+      sum[j] = j < q.partials ? n[j] * v[j].x : 0.0;
+    }
+    const double mu = ((sum[0] + sum[2]) + (sum[1] + sum[3])) / (double)p.count;
+#pragma unroll
+    for (unsigned j = 0; j < kWhole; ++j) dev[j] = j < q.partials ? v[j].y + n[j] * (v[j].x - mu) * (v[j].x - mu) : 0.0;
+    m = (float)mu;
+    rs = 1.0f / sqrtf((float)(((dev[0] + dev[2]) + (dev[1] + dev[3])) / (double)p.count) + q.eps);
+  }
+}
+
 // STREAM: loads and stores that leave nothing in the last-level cache, for tensors that do not fit there
-template <int DT, bool BWD, bool STREAM>
-__global__ __launch_bounds__(kThreads, 4) void gn_resident_kernel(ResidentArgs q, ApplyArgs p) {
+// WHOLE: a block has a part of kThreads threads for each chunk of its unit (blockIdx.x), up to kWhole of them: the partials meet in LDS,
+// nobody waits for another block, and neither the words nor the list are wanted. One launch forward where there are three,
+// two backward: a short step is bound by the host, which takes 3 to 4 us a launch (forward and backward of 4 x 64 x 259 x 83 bf16 in
+// 32 groups and of smaller tensors, us: 78 with six launches, 66 with three)
+template <int DT, bool BWD, bool STREAM, bool WHOLE>
+__global__ __launch_bounds__(WHOLE ? kWhole * kThreads : kThreads, 4) void gn_resident_kernel(ResidentArgs q, ApplyArgs p) {
   typedef typename Elem<DT>::T T;
   constexpr int V = Elem<DT>::VEC, E = 4 / sizeof(T), R = kHeld<BWD>, kAux = STREAM ? 2 : 0;  // 2: non-temporal
-  const int tid = threadIdx.x;
+  constexpr int PARTS = WHOLE ? kWhole : 1;
+  const int tid = threadIdx.x % kThreads;
+  const unsigned me = WHOLE ? blockIdx.x * q.partials + __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads) : blockIdx.x;
   const T* in = static_cast<const T*>(p.in);
   const T* in2 = static_cast<const T*>(p.in2);
-  const HeldRange r = held_range(q, p, blockIdx.x);
+  const HeldRange r = held_range(q, p, me);
   float m = BWD ? q.mean[r.unit] : 0.0f, rs, q1, q2;
 
   // the chunk into registers: whole vectors, and the elements before the first and behind the last one, one a thread
@@ -660,7 +707,7 @@ __global__ __launch_bounds__(kThreads, 4) void gn_resident_kernel(ResidentArgs q
     }
     part.x += sa;
     part.y += sa * (sb - m);
-    part = block_total2(part.x, part.y);
+    part = block_total2<PARTS>(part.x, part.y);
     part.y *= q.rstd[r.unit];
   } else {
     const float n = (float)(r.hi - r.lo);
@@ -671,7 +718,8 @@ __global__ __launch_bounds__(kThreads, 4) void gn_resident_kernel(ResidentArgs q
 #pragma unroll
       for (int e = 0; e < V; ++e) sum += up_of<DT>(a[i][e / E], e % E);
     }
-    part.x = n > 0.0f ? block_total(sum) / n : 0.0f;
+    const float all = block_total<float, PARTS>(sum);
+    part.x = n > 0.0f ? all / n : 0.0f;
     float dev = has_single ? (sa - part.x) * (sa - part.x) : 0.0f;
 #pragma unroll
     for (int i = 0; i < R; ++i)
@@ -681,30 +729,38 @@ __global__ __launch_bounds__(kThreads, 4) void gn_resident_kernel(ResidentArgs q
           const float d = up_again<DT>(a[i][e / E], e % E) - part.x;
           dev += d * d;
         }
-    part.y = block_total(dev);
+    part.y = block_total<float, PARTS>(dev);
   }
-  if (tid == 0) publish(q.slot + blockIdx.x, part.x, part.y);
-
-  __shared__ unsigned long long word_s;
-  const bool adds = q.partials <= kDirect || r.k == q.partials - 1;
-  const unsigned gave_up = __hip_atomic_load(q.left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const unsigned polls = gave_up > (blockIdx.x + q.partials) / 2 && q.polls > kPollsStarved ? kPollsStarved : q.polls;
-  bool there;
-  if (adds) {
-    there = held_statistics<DT, BWD>(q, p, r.unit, polls, m, rs, q1, q2);
-    if (there && tid == 0 && q.partials > kDirect) publish(q.result + r.unit, BWD ? q1 : m, BWD ? q2 : rs);
-  } else {
-    if (tid == 0) word_s = await(q.result + r.unit, polls);
+  if (WHOLE) {
+    __shared__ float2 parts[kWhole];
+    if (tid == 0) parts[r.k] = part;
+    if (BWD && tid == 0) publish(q.slot + me, part.x, part.y);  // for the parameter gradients
     __syncthreads();
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)word_s), hi = __builtin_amdgcn_readfirstlane((unsigned)(word_s >> 32));
-    there = (lo & hi) != ~0u;
-    const float v0 = __uint_as_float(lo), v1 = __uint_as_float(hi);
-    if (BWD) q1 = v0, q2 = v1, rs = q.rstd[r.unit];
-    else m = v0, rs = v1;
-  }
-  if (!there) {
-    if (tid == 0) q.list[__hip_atomic_fetch_add(q.left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)] = blockIdx.x;
-    return;
+    whole_statistics<DT, BWD>(q, p, r.unit, parts, m, rs, q1, q2);
+  } else {
+    if (tid == 0) publish(q.slot + blockIdx.x, part.x, part.y);
+
+    __shared__ unsigned long long word_s;
+    const bool adds = q.partials <= kDirect || r.k == q.partials - 1;
+    const unsigned gave_up = __hip_atomic_load(q.left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned polls = gave_up > (blockIdx.x + q.partials) / 2 && q.polls > kPollsStarved ? kPollsStarved : q.polls;
+    bool there;
+    if (adds) {
+      there = held_statistics<DT, BWD>(q, p, r.unit, polls, m, rs, q1, q2);
+      if (there && tid == 0 && q.partials > kDirect) publish(q.result + r.unit, BWD ? q1 : m, BWD ? q2 : rs);
+    } else {
+      if (tid == 0) word_s = await(q.result + r.unit, polls);
+      __syncthreads();
+      const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)word_s), hi = __builtin_amdgcn_readfirstlane((unsigned)(word_s >> 32));
+      there = (lo & hi) != ~0u;
+      const float v0 = __uint_as_float(lo), v1 = __uint_as_float(hi);
+      if (BWD) q1 = v0, q2 = v1, rs = q.rstd[r.unit];
+      else m = v0, rs = v1;
+    }
+    if (!there) {
+      if (tid == 0) q.list[__hip_atomic_fetch_add(q.left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)] = blockIdx.x;
+      return;
+    }
   }
   if (!BWD && r.k == 0 && tid == 0) {
     q.mean[r.unit] = m;
@@ -737,7 +793,7 @@ __global__ __launch_bounds__(kThreads, 4) void gn_resident_kernel(ResidentArgs q
 }
 
 // Behind gn_resident_kernel: the parameter gradients of channel blockIdx.x from its rows' partials of every sample
-// (backward, blocks [0, C) if they are wanted), and the chunks on the list, one block after the other.
+// (backward, blocks [0, C) if they are wanted), and the chunks on the list, if there is one, one block after the other.
 template <int DT, bool BWD>
 __global__ __launch_bounds__(kThreads) void gn_resident_rest_kernel(ResidentArgs q, ApplyArgs p, void* gw, void* gb, int wdtype, long long N) {
   const int tid = threadIdx.x;
@@ -754,7 +810,7 @@ __global__ __launch_bounds__(kThreads) void gn_resident_rest_kernel(ResidentArgs
     if (tid == 0 && gb != nullptr) store_as(gb, c, sums.x, wdtype);
     if (tid == 0 && gw != nullptr) store_as(gw, c, sums.y, wdtype);
   }
-  const unsigned left = *q.left;
+  const unsigned left = q.left != nullptr ? *q.left : 0;
   for (unsigned i = blockIdx.x; i < left; i += gridDim.x) {
     const HeldRange r = held_range(q, p, q.list[i]);
     float m, rs, q1, q2;
@@ -886,13 +942,20 @@ bool resident_launch(ResidentArgs q, const ApplyArgs& a, void* gw, void* gb, int
   q.partials = (unsigned)(cpg * chunks);
   q.S = S;
   q.chunk_len = chunk_len_of(S, (int)chunks);
+  const long long channels = gw != nullptr || gb != nullptr ? a.C : 0, bytes = rows * S * (long long)sizeof(typename Elem<DT>::T);
+  // A unit of up to kWhole chunks is one block's. (Not for `polls` of a test's own.)
+  if (q.partials <= kWhole && q.polls == kPolls && bytes < kStreamed) {
+    gn_resident_kernel<DT, BWD, false, true><<<(unsigned)units, kThreads * q.partials, 0, s>>>(q, a);
+    q.left = nullptr;
+    if (channels > 0) gn_resident_rest_kernel<DT, BWD><<<(unsigned)channels, kThreads, 0, s>>>(q, a, gw, gb, wdtype, N);
+    return true;
+  }
   gn_resident_clear_kernel<<<(unsigned)((total + units + kThreads - 1) / kThreads), kThreads, 0, s>>>(q.slot, q.left, total + units);
   // Two tensors that fill the last-level cache (256 MB) go past it; smaller ones stay for whoever reads them next. Forward and
   // backward: 8 x 32 x 512^2 bf16 (134 MB) 155 us against 170, 8 x 64 x 1024^2 1159 against 1262; 4 x 64 x 300 x 311 fp32
   // (95 MB) 153 against 135.
-  if (rows * S * (long long)sizeof(typename Elem<DT>::T) >= 1ll << 27) gn_resident_kernel<DT, BWD, true><<<(unsigned)total, kThreads, 0, s>>>(q, a);
-  else gn_resident_kernel<DT, BWD, false><<<(unsigned)total, kThreads, 0, s>>>(q, a);
-  const long long channels = gw != nullptr || gb != nullptr ? a.C : 0;
+  if (bytes >= kStreamed) gn_resident_kernel<DT, BWD, true, false><<<(unsigned)total, kThreads, 0, s>>>(q, a);
+  else gn_resident_kernel<DT, BWD, false, false><<<(unsigned)total, kThreads, 0, s>>>(q, a);
   gn_resident_rest_kernel<DT, BWD><<<(unsigned)std::max(channels, std::min(total, fit)), kThreads, 0, s>>>(q, a, gw, gb, wdtype, N);
   return true;
 }

@@ -304,6 +304,20 @@ def test_the_launch_that_writes_a_chunk_does_not_show(shape, dtype, dev):
             assert torch.equal(t, want[name]), f"{name} at {polls} polls"
 
 
+@pytest.mark.parametrize("shape", [
+    # batch, channels, groups, positions: the edges of a block that keeps a whole group, forward (4 x 32768 16-bit elements) and backward (half of it)
+    (1, 1, 1, 1), (3, 6, 2, 7), (2, 4, 1, 16384), (2, 8, 2, 16385), (1, 2, 1, 32768), (5, 2, 1, 32769), (1, 1, 1, 4 * 16384 - 1), (1, 2, 2, 4 * 16384 + 9),
+    (2, 3, 1, 32767), (1, 1, 1, 4 * 32768), (1, 5, 1, 100), (9, 32, 32, 211),
+], ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_a_group_that_one_block_keeps_has_the_bits_of_several(shape, dtype, dev):
+    """The default call (128 polls), where small groups meet in LDS, and the same with blocks that wait for each other."""
+    run = _whole_tensor(shape, dtype, dev)
+    got, want = run(128), run(256)
+    for name, t in got.items():
+        assert not t.isnan().any() and torch.equal(t, want[name]), name
+
+
 def test_a_busy_chip_does_not_show_in_the_results(dev):
     """Beside a kernel of another stream that keeps four fifths of the compute units, where blocks do give up, bit for bit what
     the same call gives alone; and again on the free chip after it."""
