@@ -641,7 +641,11 @@ int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
   // 2048 queries x 4 chunks 94 : 81, 3 x 4000 x 8 321 : 285, 18 x 700 x 3 32 : 26. Elsewhere twice the tile
   // traffic and a barrier for half the keys cost more than the waves' independence gives: 8 x 4096 x 4 203 : 223, 32 x 1024 x 1
   // 18.0 : 18.9, 24 x 1000 x 2 30.8 : 32.1.
+  // And there dQ, dK and dV in one launch where attn_wide.hip takes that to be the shorter way (two launches : one, us; fp16 for the latter): 7 x 387 x 6 chunks
+  // 35.2 : 27.3, 15 x 313 x 7 42.9 : 31.6, 6 x 400 x 4 25.8 : 20.2.
   if (attn_width(sq, batch, D) == 1) {
+    if (attn_wide_bwd_one_launch(batch, sq, sk, nchunks))
+      return attn_wide_bwd_chunks(dq, dk, dv, dout, q, k, v, nchunks, out, lse, batch, sq, sk, D, JG_BF16, scale, ws, s);
     const int rc = attn_wide_bwd_chunks(dq, nullptr, nullptr, dout, q, k, v, nchunks, out, lse, batch, sq, sk, D, JG_BF16, scale, ws, s);
     if (rc != JG_OK) return rc;
   } else if (2 * batch * cdiv(sq, DqPlan<4>::ROWS) <= cu_count()) launch_dq(std::integral_constant<int, 2>{});

@@ -97,6 +97,7 @@ int attn_wide_fwd_chunks(void* out, float* lse, const void* q, const void* const
 int attn_wide_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q, const void* const* k,
                          const void* const* v, int nchunks, const void* out, const float* lse, long long batch, int sq,
                          int sk, int d, int dtype, float scale, void* ws, hipStream_t s);
+bool attn_wide_bwd_one_launch(long long batch, int sq, int sk, int nchunks);  // whether that forms dQ, dK and dV of heads of 64 in one launch
 
 // Workgroup -> (batch entry, chunk, row block) of a grid (row blocks, batch entries, chunks). Consecutive
 // workgroup ids go to the 8 XCDs in turn; each XCD is given a contiguous range of the flat order (batch entry,
@@ -107,9 +108,7 @@ struct BlockOf {
   int blk;
   int chunk;
 };
-__device__ __forceinline__ BlockOf block_of() {
-  const unsigned nblk = gridDim.x, nch = gridDim.z, total = gridDim.x * gridDim.y * gridDim.z;
-  unsigned id = (blockIdx.y * nch + blockIdx.z) * nblk + blockIdx.x;
+__device__ __forceinline__ BlockOf block_at(unsigned id, unsigned total, unsigned nblk, unsigned nch) {
   if ((total & 7u) == 0) id = (id & 7u) * (total >> 3) + (id >> 3);
   BlockOf b;
   b.blk = (int)(id % nblk);
@@ -117,6 +116,10 @@ __device__ __forceinline__ BlockOf block_of() {
   b.chunk = (int)(id % nch);
   b.bh = id / nch;
   return b;
+}
+__device__ __forceinline__ BlockOf block_of() {
+  const unsigned nblk = gridDim.x, nch = gridDim.z;
+  return block_at((blockIdx.y * nch + blockIdx.z) * nblk + blockIdx.x, gridDim.x * gridDim.y * gridDim.z, nblk, nch);
 }
 
 }  // namespace jg

@@ -77,6 +77,7 @@ struct Geo {
   __device__ static __forceinline__ int swizzle(int r) { return ((r >> 2) & 3) | (D == 64 ? ((r >> 1) & 1) << 2 : (D == 128 ? (r & 3) << 2 : 0)); }
   static constexpr int RV = D == 64 ? 4 : (D == 128 ? 8 : 2), TV = RV / 2;  // pieces, and blocks of 32 columns, whose swizzles differ
   static constexpr int CHUNKS = BT * D / 8;  // 16-byte pieces of a tile
+  static constexpr int DOTS = D == 96 ? 3 : 1;  // sums that a row's dot product comes in (tile_row_dots)
 };
 
 template <int D, int W>
@@ -113,6 +114,11 @@ __device__ __forceinline__ void tile_store(const TileRegs<D, W>& r, unsigned cha
     }
   }
 }
+
+// dots[row] = sum over the columns of a b for the rows of two fetched tiles, zero for rows and without columns that do not exist. The lanes of a
+// row's pieces lie behind each other: a tree over them, or, 12 of them, over each four: three sums, dots[32 i + row].
+template <int D, bool F16, int W>
+__device__ __forceinline__ void tile_row_dots(const TileRegs<D, W>& a, const TileRegs<D, W>& b, float* dots, int tid, int d);
 
 __device__ __forceinline__ f32x16 zero16() {
   f32x16 z;
@@ -158,6 +164,28 @@ struct Half<true> {
 template <bool F16>
 __device__ __forceinline__ typename Half<F16>::x8 frag(const unsigned char* at) {
   return __builtin_bit_cast(typename Half<F16>::x8, *reinterpret_cast<const u32x4*>(at));
+}
+template <int D, bool F16, int W>
+__device__ __forceinline__ void tile_row_dots(const TileRegs<D, W>& a, const TileRegs<D, W>& b, float* dots, int tid, int d) {
+  constexpr int PIECES = D / 8, TREE = PIECES / Geo<D>::DOTS;
+  static_assert((TREE & (TREE - 1)) == 0, "a power of two");
+#pragma unroll
+  for (int i = 0; i < TileRegs<D, W>::PER; ++i) {
+    const int c = tid + i * (W * 64), row = c / PIECES, piece = c % PIECES;
+    float sum = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float a0, a1, b0, b1;
+      Half<F16>::unpair(a.v[i][e], a0, a1);
+      Half<F16>::unpair(b.v[i][e], b0, b1);
+      sum = __builtin_fmaf(a0, b0, sum);
+      sum = __builtin_fmaf(a1, b1, sum);
+    }
+    sum = row < a.rows && piece * 8 < d ? sum : 0.0f;
+#pragma unroll
+    for (int o = 1; o < TREE; o <<= 1) sum += __shfl_xor(sum, o, 64);
+    if (piece % TREE == 0 && c < Geo<D>::CHUNKS) dots[piece / TREE * BT + row] = sum;
+  }
 }
 // Where a lane finds its parts of a tile: fragments of row ln (columns 16 c + 8 kg + 0..7), and transposed ones by LDS transpose reads (within
 // 16 lanes, lane i receives element i % 4 of the 8 bytes that lanes i / 4 + 4 j point at, j = 0..3): lane (ln, kg) gets column ln of
@@ -264,7 +292,7 @@ struct Args {
   const uint16_t* out;   // backward: the global output
   const uint16_t* dout;  // backward
   const float* lse_in;   // backward: the global lse
-  float* delta;          // backward workspace (batch, sq): written by the dQ kernel, read by the dK/dV kernel
+  float* delta;          // backward workspace (batch, sq): written by the dQ kernel, read by the dK/dV kernel (not where they are one launch)
   uint16_t* o;           // forward output, or NULL when only the merge is wanted
   float* lse;            // forward output, or NULL
   float* out_acc;        // forward: fp32 (batch, sq, d) accumulator of the ring, merged in place, or NULL
@@ -499,8 +527,9 @@ __device__ __forceinline__ void hand_over(float* lds, int ks, int wave, int lane
 
 // ------------------------------------------------------------------- dQ (and delta)
 // EXACT (here and in the dK/dV kernel): dS and the probabilities are not rounded (chunks of fewer than EXACT_KEYS keys).
-template <int D, bool F16, int W, int KS, bool EXACT>
-__global__ __launch_bounds__(64 * W * KS) void attn_wide_dq_kernel(ChunkTable, Args p) {
+// STORE: delta goes to the workspace for a dK/dV launch.
+template <int D, bool F16, int W, int KS, bool EXACT, bool STORE>
+__device__ __forceinline__ void dq_block(const Args& p, const BlockOf& wg) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
   constexpr int BUF = 2 * G::TILE;  // K tile, V tile
@@ -508,7 +537,6 @@ __global__ __launch_bounds__(64 * W * KS) void attn_wide_dq_kernel(ChunkTable, A
   const int tid = threadIdx.x % (64 * W), ks = threadIdx.x / (64 * W);
   const int lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kg = lane >> 5;
-  const BlockOf wg = block_of();
   const long long bh = wg.bh;
   const bool live = wg.blk * (32 * W) + wave * 32 + ln < p.sq;
   const int qi = live ? wg.blk * (32 * W) + wave * 32 + ln : p.sq - 1;
@@ -530,7 +558,7 @@ __global__ __launch_bounds__(64 * W * KS) void attn_wide_dq_kernel(ChunkTable, A
   }
   // delta = rowsum(dO o O): the two lanes of a query hold disjoint halves of the row
   const float delta = dl + __shfl_xor(dl, 32, 64);
-  if (kg == 0 && ks == 0 && live) p.delta[bh * p.sq + qi] = delta;
+  if (STORE && kg == 0 && ks == 0 && live) p.delta[bh * p.sq + qi] = delta;
   const float lse2 = p.lse_in[bh * p.sq + qi] * LOG2E;
 
   f32x16 dq[G::NB];
@@ -617,31 +645,37 @@ __global__ __launch_bounds__(64 * W * KS) void attn_wide_dq_kernel(ChunkTable, A
     }
 }
 
+template <int D, bool F16, int W, int KS, bool EXACT>
+__global__ __launch_bounds__(64 * W * KS) void attn_wide_dq_kernel(ChunkTable, Args p) {
+  dq_block<D, F16, W, KS, EXACT, true>(p, block_of());
+}
+
 // ------------------------------------------------------------------- dK, dV
 // MODE 0 forms dK and dV in one pass (two d x 32 accumulators a wavefront). That fits two workgroups
 // per CU in 256 registers a lane at head size 96 but not at 128 (it would spill, and ran 1.3x slower
 // that way), so head sizes above 96 run the kernel twice: MODE 1 forms dV only (from P), MODE 2 dK only
 // (from dS), each with one accumulator and two workgroups per CU; the scores are computed in both.
 // A launch with no more workgroups than CUs gains nothing from that and keeps the single pass.
-template <int D, bool F16, int MODE, int W, int KS, bool EXACT>
-__global__ __launch_bounds__(64 * W * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 : 1) void attn_wide_dkv_kernel(ChunkTable, Args p) {
+// OWN: delta of a tile's queries from its rows of O and dO, which are here for it, and not from a dQ launch before.
+template <int D, bool F16, int MODE, int W, int KS, bool EXACT, bool OWN>
+__device__ __forceinline__ void dkv_block(const Args& p, const BlockOf& wg) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
   constexpr bool DV = MODE != 2, DK = MODE != 1;
-  constexpr int STATS = 2 * BT * 4;                           // lse * log2(e) and delta of the tile's queries
+  constexpr int STATS = (1 + (OWN ? G::DOTS : 1)) * BT * 4;   // lse * log2(e) and delta of the tile's queries
   constexpr int BUF = 2 * G::TILE + STATS;                    // Q tile, dO tile, stats
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x % (64 * W), ks = threadIdx.x / (64 * W);
   const int lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kg = lane >> 5;
-  const BlockOf wg = block_of();
   const long long bh = wg.bh;
   const bool live = wg.blk * (32 * W) + wave * 32 + ln < p.sk;
   const long long koff = (bh * p.sk + (live ? wg.blk * (32 * W) + wave * 32 + ln : p.sk - 1)) * p.d;
   const uint16_t* qb = p.q + bh * p.sq * p.d;
   const uint16_t* gb = p.dout + bh * p.sq * p.d;
   const float* lb = p.lse_in + bh * p.sq;
-  const float* db = p.delta + bh * p.sq;
+  const float* db = OWN ? lb : p.delta + bh * p.sq;
+  const uint16_t* ob = OWN ? p.out + bh * p.sq * p.d : nullptr;
   const float c2 = p.scale * LOG2E;
   unsigned char* lds = smem + ks * 2 * BUF;
   const TileView<D, F16> view(lane);
@@ -663,7 +697,7 @@ __global__ __launch_bounds__(64 * W * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 
     if (DV) dv[nb] = zero16();
   }
 
-  TileRegs<D, W> rq, rg;
+  TileRegs<D, W> rq, rg, ro;
   float st = 0.0f;  // one statistic per thread of the group's first wavefront: lse2 (lanes 0-31) or delta (32-63)
   int st_rows = 0;  // rows of the tile it belongs to
   Stream<KS> load(0, p.sq, ks);
@@ -673,6 +707,7 @@ __global__ __launch_bounds__(64 * W * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 
     const int rows = load.rows_left();
     tile_fetch<D, W>(rq, qb + at, tid, rows, p.d);
     tile_fetch<D, W>(rg, gb + at, tid, rows, p.d);
+    if (OWN) tile_fetch<D, W>(ro, ob + at, tid, rows, p.d);
     if (tid < 2 * BT) {
       const float* src = tid < BT ? lb : db;  // every lane loads; the factor is applied when stored
       st = src[min(load.first_row() + (tid & (BT - 1)), p.sq - 1)];
@@ -687,8 +722,9 @@ __global__ __launch_bounds__(64 * W * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 
     if (tid < 2 * BT) {
       float v = tid < BT ? st * LOG2E : st;
       if ((tid & (BT - 1)) >= st_rows) v = tid < BT ? INFINITY : 0.0f;  // a query past the end: probability 0
-      reinterpret_cast<float*>(base + 2 * G::TILE)[tid] = v;
+      if (!OWN || tid < BT) reinterpret_cast<float*>(base + 2 * G::TILE)[tid] = v;
     }
+    if constexpr (OWN) tile_row_dots<D, F16, W>(rg, ro, reinterpret_cast<float*>(base + 2 * G::TILE) + BT, tid, p.d);
   };
   fetch();
   store(0);
@@ -716,7 +752,11 @@ __global__ __launch_bounds__(64 * W * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 
     for (int j = 0; j < 4; ++j) {
       const f32x4 l4 = *reinterpret_cast<const f32x4*>(stats + 8 * j + 4 * kg);
       f32x4 d4 = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (DK) d4 = *reinterpret_cast<const f32x4*>(stats + BT + 8 * j + 4 * kg);
+      if (DK) {
+        d4 = *reinterpret_cast<const f32x4*>(stats + BT + 8 * j + 4 * kg);
+#pragma unroll
+        for (int i = 1; i < (OWN ? G::DOTS : 1); ++i) d4 += *reinterpret_cast<const f32x4*>(stats + (1 + i) * BT + 8 * j + 4 * kg);
+      }
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int i = 4 * j + e;
@@ -788,6 +828,20 @@ __global__ __launch_bounds__(64 * W * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 
     }
 }
 
+template <int D, bool F16, int MODE, int W, int KS, bool EXACT>
+__global__ __launch_bounds__(64 * W * KS, KS == 1 && (D <= 96 || MODE != 0) ? 2 : 1) void attn_wide_dkv_kernel(ChunkTable, Args p) {
+  dkv_block<D, F16, MODE, W, KS, EXACT, false>(p, block_of());
+}
+
+// ------------------------------------------------------------------- dQ, dK and dV in one launch
+// The first dq_blocks workgroups form dQ, the others dK and dV, with delta of their own (see one_launch_width).
+template <int D, bool F16, int W, bool EXACT>
+__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_wide_bwd_kernel(ChunkTable, Args p, unsigned dq_blocks, unsigned q_rows, unsigned k_rows) {
+  const unsigned rest = gridDim.x - dq_blocks;
+  if (blockIdx.x < dq_blocks) dq_block<D, F16, W, 4 / W, EXACT, false>(p, jg::block_at(blockIdx.x, dq_blocks, q_rows, 1));
+  else dkv_block<D, F16, 0, W, 4 / W, EXACT, true>(p, jg::block_at(blockIdx.x - dq_blocks, rest, k_rows, p.nchunks));
+}
+
 // Workgroups of 128 rows (attn_width: half of the CUs and more have one; at head size 32 all of them, twice): where some CU has none, two
 // groups share the streamed side.
 bool two_groups(long long workgroups) { return workgroups < jg::cu_count(); }
@@ -808,6 +862,27 @@ typedef std::integral_constant<int, 2> Two;
 typedef std::integral_constant<int, 4> Four;
 template <int D>
 using Most = std::integral_constant<int, D <= 64 ? 8 : 4>;  // groups of one wavefront each whose stages LDS holds
+
+// Wavefronts that share a tile and groups of them, by kernel
+struct Shape {
+  int w, ks;
+};
+template <int D>
+Shape dq_shape(const Args& a, long long batch) {
+  switch (jg::attn_width(a.sq, batch, D)) {
+    case 1: return {1, Most<D>::value};
+    case 2: return {2, 4};
+  }
+  return {4, D > 32 && two_groups(jg::cdiv(a.sq, 128) * batch) ? 2 : 1};
+}
+template <int D>
+Shape dkv_shape(const Args& a, long long batch) {
+  switch (jg::attn_width(a.sk, batch * a.nchunks, D)) {  // (four wavefronts: a head of 128 then has the registers for both sums)
+    case 1: return {1, 4};
+    case 2: return {2, 2};
+  }
+  return {4, D > 32 && D <= 96 && two_groups(jg::cdiv(a.sk, 128) * batch * a.nchunks) ? 2 : 1};
+}
 
 template <int D, bool F16, bool EXACT>
 int launch_fwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
@@ -838,12 +913,11 @@ int launch_dq(const ChunkTable& tab, const Args& a, long long batch, hipStream_t
     return launch(&attn_wide_dq_kernel<D, F16, W, KS, EXACT>, dim3((unsigned)jg::cdiv(a.sq, 32 * W), (unsigned)batch, 1), 64 * W * KS,
                   std::max(STAGES, SUMS), tab, a, s, "jg_attn_bwd(wide, dq)");
   };
-  switch (jg::attn_width(a.sq, batch, D)) {
-    case 1: return go(One{}, Most<D>{});
-    case 2: return go(Two{}, Four{});
-  }
+  const Shape shape = dq_shape<D>(a, batch);
+  if (shape.w == 1) return go(One{}, Most<D>{});
+  if (shape.w == 2) return go(Two{}, Four{});
   if constexpr (D > 32)
-    if (two_groups(jg::cdiv(a.sq, 128) * batch)) return go(Four{}, Two{});
+    if (shape.ks == 2) return go(Four{}, Two{});
   return go(Four{}, One{});
 }
 
@@ -860,21 +934,88 @@ int launch_dkv(const ChunkTable& tab, const Args& a, long long batch, hipStream_
   };
   typedef std::integral_constant<int, 0> Both;
   const long long workgroups = jg::cdiv(a.sk, 128) * batch * a.nchunks;
-  switch (jg::attn_width(a.sk, batch * a.nchunks, D)) {  // (four wavefronts: a head of 128 then has the registers for both sums)
-    case 1: return go(Both{}, One{}, Four{});
-    case 2: return go(Both{}, Two{}, Two{});
-  }
+  const Shape shape = dkv_shape<D>(a, batch);
+  if (shape.w == 1) return go(Both{}, One{}, Four{});
+  if (shape.w == 2) return go(Both{}, Two{}, Two{});
   // up to head size 96 (64 with EXACT): dK and dV in one pass; above: one pass each when the launch has more workgroups
   // than the chip has CUs, and with EXACT always (register budget, see the kernel)
   if constexpr (D <= (EXACT ? 64 : 96)) {
     if constexpr (D > 32)
-      if (two_groups(workgroups)) return go(Both{}, Four{}, Two{});
+      if (shape.ks == 2) return go(Both{}, Four{}, Two{});
   } else if (EXACT || workgroups > jg::cu_count()) {
     const int rc = go(One{}, Four{}, One{});
     return rc != JG_OK ? rc : go(Two{}, Four{}, One{});
   }
   if constexpr (D <= 64 || !EXACT) return go(Both{}, Four{}, One{});
   return JG_OK;
+}
+
+// ---- dQ, dK and dV in one launch, or in two. Two launches one after the other each leave the compute units idle that their own workgroups do
+// not fill or that wait for the last of them, and a short step waits for the host's second launch; in one launch the two kinds fill the
+// chip together, for delta computed again by every dK/dV workgroup.
+// Up to 64 columns both ways are priced in steps of a workgroup of four wavefronts (about 0.45 us at 32 columns, 0.75 at 64): a compute unit makes
+// one at a time, 1.1 of them where it has a workgroup alone, and one of eight wavefronts takes 1.8 and 2. In one launch a head of 64 columns takes 1.25 (its
+// registers let two workgroups on a compute unit), and workgroups of 32 rows, which fetch a tile for one wavefront each, 1.2 and 1.7. A launch more is
+// six steps. Taken where one launch is expected to need less than 0.8 of the two. Backward, two launches : one, us: 4 heads x 128 x 2 chunks at 32
+// 11.3 : 7.7, 15 x 710 x 3 at 32 38.6 : 24.2, 3 x 1497 x 2 at 32 30.1 : 20.4, 16 x 802 x 3 at 32 41.7 : 31.6, 3 x 3000 x 4 at 32 140 : 100, 64 x 64 x 1 at 64
+// 14.6 : 7.1, 48 x 69 x 3 at 64 22.0 : 14.2, 15 x 313 x 7, fp16 64 42.9 : 31.6, 7 x 387 x 6, fp16 64 36.5 : 27.3. Where it says no: 8 x 1024 x 8 at 32
+// 59.0 : 61.5, 24 x 1000 x 2, fp16 64 71.7 : 74.7.
+// Wider heads have one workgroup of the one launch on a compute unit: it is taken where all of them fit at once, priced in us by what a step took
+// there, by rows, with nine for a launch and what surrounds it. 13 x 102 x 2 at 128 21.8 : 12.7, 7 x 265 x 1 at 128 26.5 : 19.7, 2 x 2000 x 2 at 128
+// 119 : 93, 2 x 1000 x 3 at 96 52.3 : 33.0, 16 x 200 x 3 at 96 23.4 : 15.4, 40 x 90 x 4 at 80 27.4 : 19.2, 1 x 2500 x 2 at 96 92 : 66. Where it says no: 12 x 1180 x 1
+// at 96 53.8 : 74.6, 8 x 512 x 4 at 128 56.8 : 61.5, 33 x 193 x 3 at 128 40.7 : 44.3 (but 30 x 140 x 4 at 128 40.8 : 34.7, more workgroups than fit).
+double steps_alone(long long workgroups, long long steps, int wavefronts) {
+  const long long each = jg::cdiv(workgroups, jg::cu_count());
+  return (wavefronts == 8 ? (each == 1 ? 1.8 : 2.0 * each) : (each == 1 ? 1.1 : 1.0 * each)) * steps;
+}
+// Rows a workgroup / 32 of the one launch (0: two launches)
+template <int D>
+int one_launch_width(const Args& a, long long batch) {
+  const int tq = jg::cdiv(a.sq, BT), tk = jg::cdiv(a.sk, BT);
+  // workgroups and steps of either kind with w wavefronts to a tile and ks groups of them
+  auto blocks_q = [&](int w) { return jg::cdiv(tq, w) * batch; };
+  auto blocks_k = [&](int w) { return jg::cdiv(tk, w) * batch * a.nchunks; };
+  auto steps_q = [&](int ks) { return (long long)jg::cdiv(tk, ks) * a.nchunks; };
+  auto steps_k = [&](int ks) { return (long long)jg::cdiv(tq, ks); };
+  const Shape q = dq_shape<D>(a, batch), k = dkv_shape<D>(a, batch);
+  int width = 0;
+  if (D <= 64) {
+    double least = 0.8 * (steps_alone(blocks_q(q.w), steps_q(q.ks), q.w * q.ks) + steps_alone(blocks_k(k.w), steps_k(k.ks), k.w * k.ks) + 6.0);
+    for (int w = 1; w <= 4; w *= 2) {
+      const double load = double(blocks_q(w) * steps_q(4 / w) + blocks_k(w) * steps_k(4 / w)) / jg::cu_count();
+      const double one = std::max(1.1 * std::max(steps_q(4 / w), steps_k(4 / w)), load * (w == 1 ? (D == 32 ? 1.2 : 1.7) : (D == 32 ? 1.0 : 1.25)));
+      if (one < least) least = one, width = w;
+    }
+    return width;
+  }
+  auto us_q = [](int w) { return w == 1 ? 1.2 : w == 2 ? 0.9 : 0.77; };
+  auto us_k = [](int w) { return w == 1 ? 3.0 : w == 2 ? 2.05 : 1.75; };
+  auto alone = [&](long long workgroups, double us, int wavefronts) { return us * (wavefronts == 8 ? 1.5 : 1.0) * jg::cdiv(workgroups, jg::cu_count()) + 9.0; };
+  double least = 0.85 * (alone(blocks_q(q.w), us_q(q.w) * steps_q(q.ks), q.w * q.ks) + alone(blocks_k(k.w), us_k(k.w) * steps_k(k.ks), k.w * k.ks));
+  for (int w = 1; w <= 4; w *= 2) {
+    const double one = std::max(us_q(w) * steps_q(4 / w), us_k(w) * steps_k(4 / w)) + 9.0;
+    if (blocks_q(w) + blocks_k(w) <= jg::cu_count() && one < least) least = one, width = w;
+  }
+  return width;
+}
+template <int D, bool F16, bool EXACT>
+int launch_bwd(const ChunkTable& tab, const Args& a, long long batch, int width, hipStream_t s) {
+  typedef Geo<D> G;
+  const char* const who = "jg_attn_bwd(wide)";
+  auto go = [&](auto w) {
+    constexpr int W = decltype(w)::value, KS = 4 / W;
+    constexpr int STAGES = KS * 2 * (2 * G::TILE + (1 + G::DOTS) * BT * 4), SUMS = KS / 2 * W * 16 * G::NB * 64 * 4, LDS = std::max(STAGES, SUMS);
+    static_assert(LDS <= 160 * 1024, "fits LDS");
+    const long long rq = jg::cdiv(a.sq, 32 * W), rk = jg::cdiv(a.sk, 32 * W), nq = rq * batch, nk = rk * batch * a.nchunks;
+    JG_REQUIRE(nq + nk < (1ll << 31), "%s: too many workgroups", who);
+    constexpr auto kernel = &attn_wide_bwd_kernel<D, F16, W, EXACT>;
+    if (LDS > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
+      JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, LDS);
+    kernel<<<(unsigned)(nq + nk), 256, LDS, s>>>(tab, a, (unsigned)nq, (unsigned)rq, (unsigned)rk);
+    JG_CHECK_LAUNCH(who);
+    return JG_OK;
+  };
+  return width == 1 ? go(One{}) : width == 2 ? go(Two{}) : go(Four{});
 }
 
 // f(D constant, F16 constant) for the narrowest kernel that holds the head. (Long bf16 sequences of narrow heads are better
@@ -891,6 +1032,12 @@ int by_width(int d, int dtype, F f) {
 }  // namespace
 
 namespace jg {
+
+bool attn_wide_bwd_one_launch(long long batch, int sq, int sk, int nchunks) {
+  Args a{};
+  a.sq = sq; a.sk = sk; a.nchunks = nchunks;
+  return one_launch_width<64>(a, batch) != 0;
+}
 
 bool attn_wide_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias) {
   return (dtype == JG_BF16 || dtype == JG_F16) && !has_bias && d > 0 && d <= 128 && d % 8 == 0 && sq > 0 && sk > 0 &&
@@ -929,6 +1076,8 @@ int attn_wide_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
   const ChunkTable tab = chunk_table(k, v, dk, dv, nchunks);
   return by_width(d, dtype, [&](auto width, auto f16) {
     const bool exact = sk < EXACT_KEYS;
+    const int rows = dk != nullptr ? one_launch_width<width()>(a, batch) : 0;
+    if (rows != 0) return exact ? launch_bwd<width(), f16(), true>(tab, a, batch, rows, s) : launch_bwd<width(), f16(), false>(tab, a, batch, rows, s);
     const int rc = exact ? launch_dq<width(), f16(), true>(tab, a, batch, s) : launch_dq<width(), f16(), false>(tab, a, batch, s);
     if (rc != JG_OK || dk == nullptr) return rc;
     return exact ? launch_dkv<width(), f16(), true>(tab, a, batch, s) : launch_dkv<width(), f16(), false>(tab, a, batch, s);
