@@ -642,9 +642,10 @@ int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
   // traffic and a barrier for half the keys cost more than the waves' independence gives: 8 x 4096 x 4 203 : 223, 32 x 1024 x 1
   // 18.0 : 18.9, 24 x 1000 x 2 30.8 : 32.1.
   // And there dQ, dK and dV in one launch where attn_wide.hip takes that to be the shorter way (two launches : one, us; fp16 for the latter): 7 x 387 x 6 chunks
-  // 35.2 : 27.3, 15 x 313 x 7 42.9 : 31.6, 6 x 400 x 4 25.8 : 20.2.
+  // 35.2 : 27.3, 15 x 313 x 7 42.9 : 31.6, 6 x 400 x 4 25.8 : 20.2. (Not for lengths in multiples of 128, where dK and dV of a chunk have the same bits in a ring
+  // and by themselves: attention.backward_chunks.)
   if (attn_width(sq, batch, D) == 1) {
-    if (attn_wide_bwd_one_launch(batch, sq, sk, nchunks))
+    if ((sq % EXACT_KEYS != 0 || sk % EXACT_KEYS != 0) && attn_wide_bwd_one_launch(batch, sq, sk, nchunks))
       return attn_wide_bwd_chunks(dq, dk, dv, dout, q, k, v, nchunks, out, lse, batch, sq, sk, D, JG_BF16, scale, ws, s);
     const int rc = attn_wide_bwd_chunks(dq, nullptr, nullptr, dout, q, k, v, nchunks, out, lse, batch, sq, sk, D, JG_BF16, scale, ws, s);
     if (rc != JG_OK) return rc;
