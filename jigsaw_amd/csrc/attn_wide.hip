@@ -320,6 +320,13 @@ struct Args {
   float scale;
 };
 
+// The larger of a lane's value and that of lane ^ 32, by a swap of registers instead of a round trip through LDS.
+__device__ __forceinline__ float pair_max(float v) {
+  const uint32_t bits = __float_as_uint(v);
+  const auto both = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+  return fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+}
+
 // ------------------------------------------------------------------- forward
 // EXACT: some keys' probabilities are not rounded (p.exact_from < p.sk). A second loop and kernels of their own: with the
 // choice inside the one loop every tile took 4 to 10 % longer, with both loops in every kernel up to 7 % (head sizes 96
@@ -327,7 +334,9 @@ struct Args {
 // What it costs, forward / backward of 64 heads x 100 queries x 8 chunks of 100 keys, rounded -> not: bf16, head size 64
 // 33 / 52 -> 34 / 58 us, 96 34 / 62 -> 40 / 78, 128 (127 keys) 35 / 86 -> 49 / 102; fp16, whose operands go in as two parts, 64
 // 34 / 52 -> 45 / 79. The one-thread-per-row kernels, which these chunks ran before, took 1107 / 2418 us at bf16 64, eight launches each way.
-template <int D, bool F16, int W, int KS, bool EXACT>
+// QB: blocks of 32 queries a wavefront. With two, a fragment from LDS feeds two matrix instructions, and the scores and products of one block run
+// under the exponentials of the other; one block leaves both to what other wavefronts the SIMD holds.
+template <int D, bool F16, int W, int KS, bool EXACT, int QB>
 __global__ __launch_bounds__(64 * W * KS) void attn_wide_fwd_kernel(ChunkTable, Args p) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
@@ -338,22 +347,25 @@ __global__ __launch_bounds__(64 * W * KS) void attn_wide_fwd_kernel(ChunkTable, 
   const int ln = lane & 31, kg = lane >> 5;
   const BlockOf wg = block_of();
   const long long bh = wg.bh;
-  const int qi = wg.blk * (32 * W) + wave * 32 + ln;
-  const bool live = qi < p.sq;
-  const uint16_t* qrow = p.q + (bh * p.sq + (live ? qi : p.sq - 1)) * p.d;
+  const int q0 = wg.blk * (32 * W * QB) + wave * (32 * QB) + ln;  // and q0 + 32, ..
   const long long chunk_off = bh * p.sk * p.d;
   const float c2 = p.scale * LOG2E;
   unsigned char* lds = smem + ks * 2 * BUF;
   const TileView<D, F16> view(lane);
 
-  X8 qf[G::C16];
+  X8 qf[QB][G::C16];
+  f32x16 o[QB][G::NB];
+  float m[QB], l[QB];
 #pragma unroll
-  for (int c = 0; c < G::C16; ++c) qf[c] = row_frag<D, F16>(qrow, 16 * c + 8 * kg, p.d);
-
-  f32x16 o[G::NB];
+  for (int qb = 0; qb < QB; ++qb) {
+    const uint16_t* qrow = p.q + (bh * p.sq + min(q0 + 32 * qb, p.sq - 1)) * p.d;
 #pragma unroll
-  for (int nb = 0; nb < G::NB; ++nb) o[nb] = zero16();
-  float m = NO_SCORE, l = 0.0f;
+    for (int c = 0; c < G::C16; ++c) qf[qb][c] = row_frag<D, F16>(qrow, 16 * c + 8 * kg, p.d);
+#pragma unroll
+    for (int nb = 0; nb < G::NB; ++nb) o[qb][nb] = zero16();
+    m[qb] = NO_SCORE;
+    l[qb] = 0.0f;
+  }
 
 #pragma unroll
   for (int pass = 0; pass < (EXACT ? 2 : 1); ++pass) {
@@ -382,57 +394,71 @@ __global__ __launch_bounds__(64 * W * KS) void attn_wide_fwd_kernel(ChunkTable, 
     // instruction that reads them, the wait sits inside the loop, behind the tile loads every iteration has
     // just issued, and counts those too: each iteration then waited for its own prefetch.
 #pragma unroll
-    for (int c = 0; c < G::C16; ++c) asm volatile("" : "+v"(qf[c]));
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+      for (int c = 0; c < G::C16; ++c) asm volatile("" : "+v"(qf[qb][c]));
     __syncthreads();
     auto tile = [&](int t, int buf) __attribute__((always_inline)) {
       const unsigned char* kt = lds + buf * BUF;
       const unsigned char* vt = kt + G::TILE;
       if (t + 1 < ntiles) fetch();
       // S^T: lane = query ln, register i = key 8*(i/4) + 4*kg + i%4 of the tile
-      f32x16 s = zero16();
+      f32x16 s[QB];
 #pragma unroll
-      for (int c = 0; c < G::C16; ++c)
-        s = Half<F16>::mma(view.rows(kt, c), qf[c], s);
+      for (int qb = 0; qb < QB; ++qb) s[qb] = zero16();
+#pragma unroll
+      for (int c = 0; c < G::C16; ++c) {
+        const X8 kf = view.rows(kt, c);
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) s[qb] = Half<F16>::mma(kf, qf[qb][c], s[qb]);
+      }
       if (soft.rows_left() < BT) {  // wave-uniform
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (8 * (i >> 2) + 4 * kg + (i & 3) >= soft.rows_left()) s[i] = -INFINITY;
+        for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if (8 * (i >> 2) + 4 * kg + (i & 3) >= soft.rows_left()) s[qb][i] = -INFINITY;
       }
       soft.next();
-      float mx = s[0];
 #pragma unroll
-      for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float mn = fmaxf(m, mx);
-      // the maximum settles after a few tiles: rescale only when some query of the wavefront saw a larger score
-      if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {
-        const float alpha = __builtin_amdgcn_exp2f((m - mn) * c2);  // first tile: 0
-        l *= alpha;
+      for (int qb = 0; qb < QB; ++qb) {
+        const f32x16& sc = s[qb];
+        // maxima of three: one instruction for two comparisons
+        auto max3 = [](float a, float b, float c) { return fmaxf(fmaxf(a, b), c); };
+        const float t0 = max3(sc[0], sc[1], sc[2]), t1 = max3(sc[3], sc[4], sc[5]), t2 = max3(sc[6], sc[7], sc[8]);
+        const float t3 = max3(sc[9], sc[10], sc[11]), t4 = max3(sc[12], sc[13], sc[14]);
+        const float mx = max3(max3(t0, t1, t2), max3(t3, t4, sc[15]), m[qb]);  // of the lane's own 16 keys and those before
+        // the maximum settles after a few tiles: the other half's keys and a rescale only when some query of the wavefront saw a larger score
+        if (__builtin_amdgcn_ballot_w64(mx > m[qb]) != 0) {
+          const float mn = pair_max(mx);
+          const float alpha = __builtin_amdgcn_exp2f((m[qb] - mn) * c2);  // first tile: 0
+          l[qb] *= alpha;
 #pragma unroll
-        for (int nb = 0; nb < G::NB; ++nb)
+          for (int nb = 0; nb < G::NB; ++nb)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) o[nb][i] *= alpha;
-        m = mn;
-      }
-      const float off = m * c2;
-      float pr[16], sum = 0.0f;
+            for (int i = 0; i < 16; ++i) o[qb][nb][i] *= alpha;
+          m[qb] = mn;
+        }
+        const float off = m[qb] * c2;
+        float pr[16], sum[2] = {0.0f, 0.0f};
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        pr[i] = __builtin_amdgcn_exp2f(s[i] * c2 - off);
-        sum += pr[i];
-      }
-      l += sum;
+        for (int i = 0; i < 16; ++i) {
+          pr[i] = __builtin_amdgcn_exp2f(sc[i] * c2 - off);
+          sum[i & 1] += pr[i];
+        }
+        l[qb] += sum[0] + sum[1];
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        if (exact) {
-          bf16x8 part[3];
-          parts8<true>(pr + 8 * ks, part);
+        for (int ks = 0; ks < 2; ++ks) {
+          if (exact) {
+            bf16x8 part[3];
+            parts8<true>(pr + 8 * ks, part);
 #pragma unroll
-          for (int nb = 0; nb < G::NB; ++nb) o[nb] = mma_exact<F16>(view.trans(vt, nb, ks), part, o[nb]);
-        } else {
-          const X8 pf = pack8<F16>(pr + 8 * ks);
+            for (int nb = 0; nb < G::NB; ++nb) o[qb][nb] = mma_exact<F16>(view.trans(vt, nb, ks), part, o[qb][nb]);
+          } else {
+            const X8 pf = pack8<F16>(pr + 8 * ks);
 #pragma unroll
-          for (int nb = 0; nb < G::NB; ++nb) o[nb] = Half<F16>::mma(view.trans(vt, nb, ks), pf, o[nb]);
+            for (int nb = 0; nb < G::NB; ++nb) o[qb][nb] = Half<F16>::mma(view.trans(vt, nb, ks), pf, o[qb][nb]);
+          }
         }
       }
       if (t + 1 < ntiles) store(buf ^ 1);
@@ -446,74 +472,86 @@ __global__ __launch_bounds__(64 * W * KS) void attn_wide_fwd_kernel(ChunkTable, 
     if (t < ntiles) tile(t, 0);
   }
   // the two lanes of a query saw the same maxima; their sums cover disjoint keys
-  l += __shfl_xor(l, 32, 64);
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) l[qb] += __shfl_xor(l[qb], 32, 64);
   if constexpr (KS > 1) {
     // the groups hand over to the one below them, halving their number each time
-    constexpr int XO = (16 * G::NB + 2) * 64;  // floats of a wavefront (in the stages' place, see launch_fwd)
+    constexpr int XB = (16 * G::NB + 2) * 64, XO = QB * XB;  // floats of 32 queries and of a wavefront (in the stages' place, see launch_fwd)
     float* xo = reinterpret_cast<float*>(smem) + ((ks % (KS / 2)) * W + wave) * XO + lane;
 #pragma unroll
     for (int half = KS / 2; half >= 1; half >>= 1) {
       if (ks >= half && ks < 2 * half) {
         float* to = reinterpret_cast<float*>(smem) + ((ks - half) * W + wave) * XO + lane;
 #pragma unroll
-        for (int nb = 0; nb < G::NB; ++nb)
+        for (int qb = 0; qb < QB; ++qb) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i) to[(nb * 16 + i) * 64] = o[nb][i];
-        to[16 * G::NB * 64] = m;
-        to[(16 * G::NB + 1) * 64] = l;
+          for (int nb = 0; nb < G::NB; ++nb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) to[qb * XB + (nb * 16 + i) * 64] = o[qb][nb][i];
+          to[qb * XB + 16 * G::NB * 64] = m[qb];
+          to[qb * XB + (16 * G::NB + 1) * 64] = l[qb];
+        }
       }
       __syncthreads();
       if (ks < half) {
-        const float m1 = xo[16 * G::NB * 64], l1 = xo[(16 * G::NB + 1) * 64];
-        const float mn = fmaxf(m, m1);
-        const float a0 = __builtin_amdgcn_exp2f((m - mn) * c2), a1 = __builtin_amdgcn_exp2f((m1 - mn) * c2);
-        l = l * a0 + l1 * a1;
-        m = mn;
 #pragma unroll
-        for (int nb = 0; nb < G::NB; ++nb)
+        for (int qb = 0; qb < QB; ++qb) {
+          const float m1 = xo[qb * XB + 16 * G::NB * 64], l1 = xo[qb * XB + (16 * G::NB + 1) * 64];
+          const float mn = fmaxf(m[qb], m1);
+          const float a0 = __builtin_amdgcn_exp2f((m[qb] - mn) * c2), a1 = __builtin_amdgcn_exp2f((m1 - mn) * c2);
+          l[qb] = l[qb] * a0 + l1 * a1;
+          m[qb] = mn;
 #pragma unroll
-          for (int i = 0; i < 16; ++i) o[nb][i] = o[nb][i] * a0 + xo[(nb * 16 + i) * 64] * a1;
+          for (int nb = 0; nb < G::NB; ++nb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[qb][nb][i] = o[qb][nb][i] * a0 + xo[qb * XB + (nb * 16 + i) * 64] * a1;
+        }
       }
       __syncthreads();
     }
     if (ks != 0) return;
   }
-  if (!live) return;
-  const bool none = l == 0.0f;  // no finite score: out 0, lse -inf, no weight in a merge (a score that is NaN makes l NaN)
-  const float inv = none ? 0.0f : 1.0f / l;
-  const float lse_j = none ? -INFINITY : m * p.scale + __logf(l);
-  const long long row = bh * p.sq + qi;
-  // Ring merge (the reference's _online_softmax_merge_): w = sigmoid(lse_j - lse), out += w (out_j - out),
-  // lse = logaddexp(lse, lse_j), with out_j rounded to the core's output dtype first as the unfused path has it.
-  float w = 0.0f;
-  if (p.out_acc != nullptr && !none) {
-    const float l_old = p.lse_acc[row];  // both lanes of the query read it before lane kg = 0 writes
-    w = 1.0f / (1.0f + __expf(l_old - lse_j));  // l_old = -inf -> 1
-    if (kg == 0) p.lse_acc[row] = fmaxf(l_old, lse_j) + log1pf(__expf(-fabsf(l_old - lse_j)));
-  }
-  if (p.lse != nullptr && kg == 0) p.lse[row] = lse_j;
-  // register i of block nb: output column nb*32 + 8*(i/4) + 4*kg + i%4
 #pragma unroll
-  for (int nb = 0; nb < G::NB; ++nb)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int dv = nb * 32 + 8 * j + 4 * kg;
-      if (dv >= p.d) continue;
-      const u32x2 h = pack4<F16>(o[nb][4 * j] * inv, o[nb][4 * j + 1] * inv, o[nb][4 * j + 2] * inv, o[nb][4 * j + 3] * inv);
-      if (p.o != nullptr) *reinterpret_cast<u32x2*>(p.o + row * p.d + dv) = h;
-      if (p.out_acc != nullptr) {
-        f32x4* dst = reinterpret_cast<f32x4*>(p.out_acc + row * p.d + dv);
-        f32x4 a = *dst;
-        float h0, h1, h2, h3;
-        Half<F16>::unpair(h.x, h0, h1);
-        Half<F16>::unpair(h.y, h2, h3);
-        a.x += w * (h0 - a.x);
-        a.y += w * (h1 - a.y);
-        a.z += w * (h2 - a.z);
-        a.w += w * (h3 - a.w);
-        *dst = a;
-      }
+  for (int qb = 0; qb < QB; ++qb) {
+    const int qi = q0 + 32 * qb;
+    if (qi >= p.sq) return;
+    const bool none = l[qb] == 0.0f;  // no finite score: out 0, lse -inf, no weight in a merge (a score that is NaN makes l NaN)
+    const float inv = none ? 0.0f : 1.0f / l[qb];
+    const float lse_j = none ? -INFINITY : m[qb] * p.scale + __logf(l[qb]);
+    const long long row = bh * p.sq + qi;
+    // Ring merge (the reference's _online_softmax_merge_): w = sigmoid(lse_j - lse), out += w (out_j - out),
+    // lse = logaddexp(lse, lse_j), with out_j rounded to the core's output dtype first as the unfused path has it.
+    float w = 0.0f;
+    if (p.out_acc != nullptr && !none) {
+      const float l_old = p.lse_acc[row];  // both lanes of the query read it before lane kg = 0 writes
+      w = 1.0f / (1.0f + __expf(l_old - lse_j));  // l_old = -inf -> 1
+      if (kg == 0) p.lse_acc[row] = fmaxf(l_old, lse_j) + log1pf(__expf(-fabsf(l_old - lse_j)));
     }
+    if (p.lse != nullptr && kg == 0) p.lse[row] = lse_j;
+    // register i of block nb: output column nb*32 + 8*(i/4) + 4*kg + i%4
+#pragma unroll
+    for (int nb = 0; nb < G::NB; ++nb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int dv = nb * 32 + 8 * j + 4 * kg;
+        if (dv >= p.d) continue;
+        const f32x16& ov = o[qb][nb];
+        const u32x2 h = pack4<F16>(ov[4 * j] * inv, ov[4 * j + 1] * inv, ov[4 * j + 2] * inv, ov[4 * j + 3] * inv);
+        if (p.o != nullptr) *reinterpret_cast<u32x2*>(p.o + row * p.d + dv) = h;
+        if (p.out_acc != nullptr) {
+          f32x4* dst = reinterpret_cast<f32x4*>(p.out_acc + row * p.d + dv);
+          f32x4 a = *dst;
+          float h0, h1, h2, h3;
+          Half<F16>::unpair(h.x, h0, h1);
+          Half<F16>::unpair(h.y, h2, h3);
+          a.x += w * (h0 - a.x);
+          a.y += w * (h1 - a.y);
+          a.z += w * (h2 - a.z);
+          a.w += w * (h3 - a.w);
+          *dst = a;
+        }
+      }
+  }
 }
 
 // The groups' sums to group 0: each hands over to the one below it, halving their number each time (in the stages' place, which a
@@ -543,7 +581,8 @@ __device__ __forceinline__ void hand_over(float* lds, int ks, int wave, int lane
 // ------------------------------------------------------------------- dQ (and delta)
 // EXACT (here and in the dK/dV kernel): dS and the probabilities are not rounded (chunks of fewer than EXACT_KEYS keys).
 // STORE: delta goes to the workspace for a dK/dV launch.
-template <int D, bool F16, int W, int KS, bool EXACT, bool STORE>
+// QB: blocks of 32 queries a wavefront, see the forward kernel.
+template <int D, bool F16, int W, int KS, bool EXACT, bool STORE, int QB = 1>
 __device__ __forceinline__ void dq_block(const Args& p, const BlockOf& wg) {
   typedef Geo<D> G;
   typedef typename Half<F16>::x8 X8;
@@ -553,32 +592,34 @@ __device__ __forceinline__ void dq_block(const Args& p, const BlockOf& wg) {
   const int lane = tid & 63, wave = tid >> 6;
   const int ln = lane & 31, kg = lane >> 5;
   const long long bh = wg.bh;
-  const bool live = wg.blk * (32 * W) + wave * 32 + ln < p.sq;
-  const int qi = live ? wg.blk * (32 * W) + wave * 32 + ln : p.sq - 1;
-  const long long qoff = (bh * p.sq + qi) * p.d;
+  const int q0 = wg.blk * (32 * W * QB) + wave * (32 * QB) + ln;  // and q0 + 32, ..
   const long long chunk_off = bh * p.sk * p.d;
   const float c2 = p.scale * LOG2E;
   unsigned char* lds = smem + ks * 2 * BUF;
   const TileView<D, F16> view(lane);
 
-  X8 qf[G::C16], dof[G::C16];
-  float dl = 0.0f;
+  X8 qf[QB][G::C16], dof[QB][G::C16];
+  float delta[QB], lse2[QB];
+  f32x16 dq[QB][G::NB];
 #pragma unroll
-  for (int c = 0; c < G::C16; ++c) {
-    qf[c] = row_frag<D, F16>(p.q + qoff, 16 * c + 8 * kg, p.d);
-    dof[c] = row_frag<D, F16>(p.dout + qoff, 16 * c + 8 * kg, p.d);
-    const X8 of = row_frag<D, F16>(p.out + qoff, 16 * c + 8 * kg, p.d);
+  for (int qb = 0; qb < QB; ++qb) {
+    const long long row = bh * p.sq + min(q0 + 32 * qb, p.sq - 1), qoff = row * p.d;
+    float dl = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) dl += (float)dof[c][j] * (float)of[j];
+    for (int c = 0; c < G::C16; ++c) {
+      qf[qb][c] = row_frag<D, F16>(p.q + qoff, 16 * c + 8 * kg, p.d);
+      dof[qb][c] = row_frag<D, F16>(p.dout + qoff, 16 * c + 8 * kg, p.d);
+      const X8 of = row_frag<D, F16>(p.out + qoff, 16 * c + 8 * kg, p.d);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) dl += (float)dof[qb][c][j] * (float)of[j];
+    }
+    // delta = rowsum(dO o O): the two lanes of a query hold disjoint halves of the row
+    delta[qb] = dl + __shfl_xor(dl, 32, 64);
+    if (STORE && kg == 0 && ks == 0 && q0 + 32 * qb < p.sq) p.delta[row] = delta[qb];
+    lse2[qb] = p.lse_in[row] * LOG2E;
+#pragma unroll
+    for (int nb = 0; nb < G::NB; ++nb) dq[qb][nb] = zero16();
   }
-  // delta = rowsum(dO o O): the two lanes of a query hold disjoint halves of the row
-  const float delta = dl + __shfl_xor(dl, 32, 64);
-  if (STORE && kg == 0 && ks == 0 && live) p.delta[bh * p.sq + qi] = delta;
-  const float lse2 = p.lse_in[bh * p.sq + qi] * LOG2E;
-
-  f32x16 dq[G::NB];
-#pragma unroll
-  for (int nb = 0; nb < G::NB; ++nb) dq[nb] = zero16();
 
   TileRegs<D, W> rk, rv;
   Stream<KS> load(0, p.sk, p.nchunks, ks), soft(0, p.sk, p.nchunks, ks);
@@ -600,38 +641,51 @@ __device__ __forceinline__ void dq_block(const Args& p, const BlockOf& wg) {
   store(0);
   // waited for once, here (see the forward kernel)
 #pragma unroll
-  for (int c = 0; c < G::C16; ++c) asm volatile("" : "+v"(qf[c]), "+v"(dof[c]));
+  for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+    for (int c = 0; c < G::C16; ++c) asm volatile("" : "+v"(qf[qb][c]), "+v"(dof[qb][c]));
   __syncthreads();
   auto tile = [&](int t, int buf) __attribute__((always_inline)) {
     const unsigned char* kt = lds + buf * BUF;
     const unsigned char* vt = kt + G::TILE;
     if (t + 1 < ntiles) fetch();
-    f32x16 s = zero16(), dp = zero16();
+    f32x16 s[QB], dp[QB];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) s[qb] = dp[qb] = zero16();
 #pragma unroll
     for (int c = 0; c < G::C16; ++c) {
-      s = Half<F16>::mma(view.rows(kt, c), qf[c], s);
-      dp = Half<F16>::mma(view.rows(vt, c), dof[c], dp);
+      const X8 kf = view.rows(kt, c);
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) s[qb] = Half<F16>::mma(kf, qf[qb][c], s[qb]);
+      const X8 vf = view.rows(vt, c);
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) dp[qb] = Half<F16>::mma(vf, dof[qb][c], dp[qb]);
     }
     if (soft.rows_left() < BT) {  // wave-uniform
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (8 * (i >> 2) + 4 * kg + (i & 3) >= soft.rows_left()) s[i] = -INFINITY;
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (8 * (i >> 2) + 4 * kg + (i & 3) >= soft.rows_left()) s[qb][i] = -INFINITY;
     }
     soft.next();
-    float ds[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) ds[i] = __builtin_amdgcn_exp2f(s[i] * c2 - lse2) * (dp[i] - delta);
+    for (int qb = 0; qb < QB; ++qb) {
+      float ds[16];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      if constexpr (EXACT) {
-        bf16x8 part[3];
-        parts8<false>(ds + 8 * ks, part);
+      for (int i = 0; i < 16; ++i) ds[i] = __builtin_amdgcn_exp2f(s[qb][i] * c2 - lse2[qb]) * (dp[qb][i] - delta[qb]);
 #pragma unroll
-        for (int nb = 0; nb < G::NB; ++nb) dq[nb] = mma_exact<F16>(view.trans(kt, nb, ks), part, dq[nb]);
-      } else {
-        const X8 dsf = pack8<F16>(ds + 8 * ks);
+      for (int ks = 0; ks < 2; ++ks) {
+        if constexpr (EXACT) {
+          bf16x8 part[3];
+          parts8<false>(ds + 8 * ks, part);
 #pragma unroll
-        for (int nb = 0; nb < G::NB; ++nb) dq[nb] = Half<F16>::mma(view.trans(kt, nb, ks), dsf, dq[nb]);
+          for (int nb = 0; nb < G::NB; ++nb) dq[qb][nb] = mma_exact<F16>(view.trans(kt, nb, ks), part, dq[qb][nb]);
+        } else {
+          const X8 dsf = pack8<F16>(ds + 8 * ks);
+#pragma unroll
+          for (int nb = 0; nb < G::NB; ++nb) dq[qb][nb] = Half<F16>::mma(view.trans(kt, nb, ks), dsf, dq[qb][nb]);
+        }
       }
     }
     if (t + 1 < ntiles) store(buf ^ 1);
@@ -644,25 +698,29 @@ __device__ __forceinline__ void dq_block(const Args& p, const BlockOf& wg) {
   }
   if (t < ntiles) tile(t, 0);
   if constexpr (KS > 1) {
-    hand_over<G::NB, W, KS>(reinterpret_cast<float*>(smem), ks, wave, lane, dq);
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) hand_over<G::NB, W, KS>(reinterpret_cast<float*>(smem), ks, wave, lane, dq[qb]);
     if (ks != 0) return;
   }
-  if (!live) return;
-  uint16_t* row = p.dq + qoff;
 #pragma unroll
-  for (int nb = 0; nb < G::NB; ++nb)
+  for (int qb = 0; qb < QB; ++qb) {
+    if (q0 + 32 * qb >= p.sq) return;
+    uint16_t* row = p.dq + (bh * p.sq + q0 + 32 * qb) * p.d;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int col = nb * 32 + 8 * j + 4 * kg;
-      if (col < p.d)
-        *reinterpret_cast<u32x2*>(row + col) = pack4<F16>(dq[nb][4 * j] * p.scale, dq[nb][4 * j + 1] * p.scale,
-                                                          dq[nb][4 * j + 2] * p.scale, dq[nb][4 * j + 3] * p.scale);
-    }
+    for (int nb = 0; nb < G::NB; ++nb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int col = nb * 32 + 8 * j + 4 * kg;
+        const f32x16& sum = dq[qb][nb];
+        if (col < p.d)
+          *reinterpret_cast<u32x2*>(row + col) = pack4<F16>(sum[4 * j] * p.scale, sum[4 * j + 1] * p.scale, sum[4 * j + 2] * p.scale, sum[4 * j + 3] * p.scale);
+      }
+  }
 }
 
-template <int D, bool F16, int W, int KS, bool EXACT>
-__global__ __launch_bounds__(64 * W * KS) void attn_wide_dq_kernel(ChunkTable, Args p) {
-  dq_block<D, F16, W, KS, EXACT, true>(p, block_of());
+template <int D, bool F16, int W, int KS, bool EXACT, int QB>
+__global__ __launch_bounds__(64 * W * KS, QB) void attn_wide_dq_kernel(ChunkTable, Args p) {
+  dq_block<D, F16, W, KS, EXACT, true, QB>(p, block_of());
 }
 
 // ------------------------------------------------------------------- dK, dV
@@ -860,6 +918,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_wide_bwd_kernel(Chu
 // Workgroups of 128 rows (attn_width: half of the CUs and more have one; at head size 32 all of them, twice): where some CU has none, two
 // groups share the streamed side.
 bool two_groups(long long workgroups) { return workgroups < jg::cu_count(); }
+bool keys_from(const Args& a, long long n) { return (long long)a.sk * a.nchunks >= n; }
 
 // `args` in a launch of `kernel` that needs more LDS than the default limit
 template <typename K>
@@ -902,38 +961,49 @@ Shape dkv_shape(const Args& a, long long batch) {
 template <int D, bool F16, bool EXACT>
 int launch_fwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
   typedef Geo<D> G;
-  auto go = [&](auto w, auto k) {
-    constexpr int W = decltype(w)::value, KS = decltype(k)::value;
-    constexpr int STAGES = KS * 2 * 2 * G::TILE, SUMS = KS / 2 * W * (16 * G::NB + 2) * 64 * 4;  // stages; what the groups hand over
+  auto go = [&](auto w, auto k, auto qb) {
+    constexpr int W = decltype(w)::value, KS = decltype(k)::value, QB = decltype(qb)::value;
+    constexpr int STAGES = KS * 2 * 2 * G::TILE, SUMS = KS / 2 * W * QB * (16 * G::NB + 2) * 64 * 4;  // stages; what the groups hand over
     static_assert(STAGES <= 160 * 1024 && SUMS <= 160 * 1024, "fits LDS");
-    return launch(&attn_wide_fwd_kernel<D, F16, W, KS, EXACT>, dim3((unsigned)jg::cdiv(a.sq, 32 * W), (unsigned)batch, 1), 64 * W * KS,
+    return launch(&attn_wide_fwd_kernel<D, F16, W, KS, EXACT, QB>, dim3((unsigned)jg::cdiv(a.sq, 32 * W * QB), (unsigned)batch, 1), 64 * W * KS,
                   std::max(STAGES, SUMS), tab, a, s, "jg_attn_fwd(wide)");
   };
   switch (jg::attn_width(a.sq, batch, D)) {
-    case 1: return go(One{}, Most<D>{});
-    case 2: return go(Two{}, Four{});
+    case 1: return go(One{}, Most<D>{}, One{});
+    case 2: return go(Two{}, Four{}, One{});
   }
-  if constexpr (D > 32)
-    if (two_groups(jg::cdiv(a.sq, 128) * batch)) return go(Four{}, Two{});
-  return go(Four{}, One{});
+  // 128 queries a workgroup, up to 64 columns: two blocks a wavefront in as many wavefronts, where the walk over the keys is long enough for the groups'
+  // hand-over. One block : two, us, in four wavefronts: 48 x 1000 x 3 chunks, fp16 64 83 : 74, 28 x 1162 x 2, fp16 64 64 : 58, 16 x 2924 x 4 at 32
+  // 242 : 191, 15 x 3241 x 6 at 32 398 : 309, 64 x 270 x 2 at 32 10.9 : 10.0; 300 x 96 x 3, fp16 64 24.6 : 27.9, 64 x 520 x 1, fp16 64 18.6 : 19.8, 600 x 64 x 1 at 32 6.7 :
+  // 7.7. In eight: 24 x 1193 x 7, fp16 64 113 : 107, 8 x 2690 x 6 210 : 189; 24 x 1000 x 2 32.7 : 33.7, 32 x 754 x 2 25.2 : 25.6. Above 64 columns there are no registers for it.
+  const bool two = two_groups(jg::cdiv(a.sq, 128) * batch);
+  if constexpr (D > 64) return two ? go(Four{}, Two{}, One{}) : go(Four{}, One{}, One{});
+  else if constexpr (D > 32) {
+    if (two) return keys_from(a, 4096) ? go(Two{}, Four{}, Two{}) : go(Four{}, Two{}, One{});
+  }
+  if constexpr (D <= 64) return keys_from(a, D == 32 ? 512 : 1024) ? go(Two{}, Two{}, Two{}) : go(Four{}, One{}, One{});
 }
 
 template <int D, bool F16, bool EXACT>
 int launch_dq(const ChunkTable& tab, const Args& a, long long batch, hipStream_t s) {
   typedef Geo<D> G;
-  auto go = [&](auto w, auto k) {
-    constexpr int W = decltype(w)::value, KS = decltype(k)::value;
+  auto go = [&](auto w, auto k, auto qb) {
+    constexpr int W = decltype(w)::value, KS = decltype(k)::value, QB = decltype(qb)::value;
     constexpr int STAGES = KS * 2 * 2 * G::TILE, SUMS = KS / 2 * W * 16 * G::NB * 64 * 4;
     static_assert(STAGES <= 160 * 1024 && SUMS <= 160 * 1024, "fits LDS");
-    return launch(&attn_wide_dq_kernel<D, F16, W, KS, EXACT>, dim3((unsigned)jg::cdiv(a.sq, 32 * W), (unsigned)batch, 1), 64 * W * KS,
+    return launch(&attn_wide_dq_kernel<D, F16, W, KS, EXACT, QB>, dim3((unsigned)jg::cdiv(a.sq, 32 * W * QB), (unsigned)batch, 1), 64 * W * KS,
                   std::max(STAGES, SUMS), tab, a, s, "jg_attn_bwd(wide, dq)");
   };
   const Shape shape = dq_shape<D>(a, batch);
-  if (shape.w == 1) return go(One{}, Most<D>{});
-  if (shape.w == 2) return go(Two{}, Four{});
-  if constexpr (D > 32)
-    if (shape.ks == 2) return go(Four{}, Two{});
-  return go(Four{}, One{});
+  if (shape.w == 1) return go(One{}, Most<D>{}, One{});
+  if (shape.w == 2) return go(Two{}, Four{}, One{});
+  // Two blocks a wavefront as in the forward, backward in all, one : two, us, four wavefronts: 14 x 3596 x 2 at 32 306 : 256, 16 x 2924 x 4 at 32 425 : 401,
+  // 28 x 1162 x 2, fp16 64 135 : 121, 8 x 4096 x 2, fp16 64 306 : 293; 64 x 500 x 2 at 32 30.6 : 31.3, 150 x 256 x 3, fp16 64 61.4 : 62.6. Eight: 8 x 2690 x 6, fp16 64 451 : 437.
+  if constexpr (D > 64) return shape.ks == 2 ? go(Four{}, Two{}, One{}) : go(Four{}, One{}, One{});
+  else if constexpr (D > 32) {
+    if (shape.ks == 2) return keys_from(a, 4096) ? go(Two{}, Four{}, Two{}) : go(Four{}, Two{}, One{});
+  }
+  if constexpr (D <= 64) return keys_from(a, 2048) ? go(Two{}, Two{}, Two{}) : go(Four{}, One{}, One{});
 }
 
 template <int D, bool F16, bool EXACT>
@@ -978,7 +1048,7 @@ int launch_dkv(const ChunkTable& tab, const Args& a, long long batch, hipStream_
 // Wider heads have one workgroup of the one launch on a compute unit: it is taken where all of them fit at once, priced in us by what a step took
 // there, by rows, with nine for a launch and what surrounds it. 13 x 102 x 2 at 128 21.8 : 12.7, 7 x 265 x 1 at 128 26.5 : 19.7, 2 x 2000 x 2 at 128
 // 119 : 93, 2 x 1000 x 3 at 96 52.3 : 33.0, 16 x 200 x 3 at 96 23.4 : 15.4, 40 x 90 x 4 at 80 27.4 : 19.2, 1 x 2500 x 2 at 96 92 : 66. Where it says no: 12 x 1180 x 1
-// at 96 53.8 : 74.6, 8 x 512 x 4 at 128 56.8 : 61.5, 33 x 193 x 3 at 128 40.7 : 44.3 (but 30 x 140 x 4 at 128 40.8 : 34.7, more workgroups than fit).
+// at 96 53.8 : 74.6, 12 x 503 x 2 at 80 30.9 : 34.3, 8 x 512 x 4 at 128 56.8 : 61.5, 33 x 193 x 3 at 128 40.7 : 44.3 (but 30 x 140 x 4 at 128 40.8 : 34.7, more workgroups than fit).
 double steps_alone(long long workgroups, long long steps, int wavefronts) {
   const long long each = jg::cdiv(workgroups, jg::cu_count());
   return (wavefronts == 8 ? (each == 1 ? 1.8 : 2.0 * each) : (each == 1 ? 1.1 : 1.0 * each)) * steps;
@@ -1006,7 +1076,7 @@ int one_launch_width(const Args& a, long long batch) {
   auto us_q = [](int w) { return w == 1 ? 1.2 : w == 2 ? 0.9 : 0.77; };
   auto us_k = [](int w) { return w == 1 ? 3.0 : w == 2 ? 2.05 : 1.75; };
   auto alone = [&](long long workgroups, double us, int wavefronts) { return us * (wavefronts == 8 ? 1.5 : 1.0) * jg::cdiv(workgroups, jg::cu_count()) + 9.0; };
-  double least = 0.85 * (alone(blocks_q(q.w), us_q(q.w) * steps_q(q.ks), q.w * q.ks) + alone(blocks_k(k.w), us_k(k.w) * steps_k(k.ks), k.w * k.ks));
+  double least = (D <= 96 ? 0.77 : 0.85) * (alone(blocks_q(q.w), us_q(q.w) * steps_q(q.ks), q.w * q.ks) + alone(blocks_k(k.w), us_k(k.w) * steps_k(k.ks), k.w * k.ks));
   for (int w = 1; w <= 4; w *= 2) {
     const double one = std::max(us_q(w) * steps_q(4 / w), us_k(w) * steps_k(4 / w)) + 9.0;
     if (blocks_q(w) + blocks_k(w) <= jg::cu_count() && one < least) least = one, width = w;

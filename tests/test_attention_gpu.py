@@ -685,6 +685,17 @@ def test_workgroups_of_every_width(h, sq, sk, P, d, dtype, dev):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("h,sq,sk,d,P", [
+    # workgroups of 128 rows on 256 compute units, up to 64 columns: two blocks of 32 rows a wavefront where the keys are many; blocks and
+    # wavefronts without a row, key groups with fewer tiles, chunks shorter than 128 keys; four wavefronts, then eight
+    (520, 1, 129, 24, 16), (520, 33, 600, 32, 1), (300, 97, 161, 32, 13), (260, 65, 2049, 64, 1), (257, 128, 100, 64, 16), (260, 33, 257, 48, 4), (300, 31, 33, 40, 3),
+    (120, 130, 4100, 64, 1), (125, 129, 293, 56, 14),
+])
+def test_workgroups_that_fill_the_chip(h, sq, sk, d, P, dtype, dev):
+    test_ring_of_any_lengths_in_one_pass(1, h, sq, sk, d, P, dtype, dev)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("h,sq,sk,d,P", [(4, 100, 100, 64, 2), (4, 300, 127, 64, 3), (3, 64, 31, 64, 1), (4, 100, 65, 40, 2), (3, 130, 97, 32, 5),
                                          (3, 130, 97, 96, 2), (3, 200, 127, 128, 2), (300, 130, 100, 80, 1)], ids=str)
 def test_short_key_ranges_keep_probabilities_in_fp32(h, sq, sk, d, P, dtype, dev):
