@@ -644,8 +644,12 @@ int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
   // And there dQ, dK and dV in one launch where attn_wide.hip takes that to be the shorter way (two launches : one, us; fp16 for the latter): 7 x 387 x 6 chunks
   // 35.2 : 27.3, 15 x 313 x 7 42.9 : 31.6, 6 x 400 x 4 25.8 : 20.2. (Not for lengths in multiples of 128, where dK and dV of a chunk have the same bits in a ring
   // and by themselves: attention.backward_chunks.)
-  if (attn_width(sq, batch, D) == 1) {
-    if ((sq % EXACT_KEYS != 0 || sk % EXACT_KEYS != 0) && attn_wide_bwd_one_launch(batch, sq, sk, nchunks))
+  // Those of 64 queries go there too where the keys are many (four groups take tiles of all chunks in turn; this kernel with 64 : that one, backward, us): 32 x 270 x 8
+  // 55.8 : 51.1, 30 x 394 x 6 65.8 : 61.4, 48 x 237 x 6 41.9 : 40.2, 4 x 2700 x 5 217 : 202; 18 x 745 x 2 35.4 : 35.9, 27 x 296 x 2 21.4 : 21.9. (Lengths in multiples of 128: not by a rule on the
+  // chunks' number, as above.)
+  const int width = attn_width(sq, batch, D);
+  if (width == 1 || (width == 2 && (sq % EXACT_KEYS != 0 || sk % EXACT_KEYS != 0) && (long long)sk * nchunks >= 2048)) {
+    if (width == 1 && (sq % EXACT_KEYS != 0 || sk % EXACT_KEYS != 0) && attn_wide_bwd_one_launch(batch, sq, sk, nchunks))
       return attn_wide_bwd_chunks(dq, dk, dv, dout, q, k, v, nchunks, out, lse, batch, sq, sk, D, JG_BF16, scale, ws, s);
     const int rc = attn_wide_bwd_chunks(dq, nullptr, nullptr, dout, q, k, v, nchunks, out, lse, batch, sq, sk, D, JG_BF16, scale, ws, s);
     if (rc != JG_OK) return rc;

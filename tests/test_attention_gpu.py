@@ -390,6 +390,12 @@ def test_query_gradient_in_workgroups_of_64_queries(heads, n, nk, P, dev):
     test_query_gradient_at_the_ends_of_its_key_tiles(heads, n, nk, P, dev)
 
 
+@pytest.mark.parametrize("heads,n,nk,P", [(100, 65, 257, 8), (100, 128, 130, 16), (60, 150, 683, 3), (60, 129, 1024, 2), (100, 70, 146, 14), (70, 97, 2047, 1)], ids=str)
+def test_query_gradient_in_workgroups_of_64_queries_over_many_keys(heads, n, nk, P, dev):
+    """Lengths that are no multiples of 128, on either side of 2048 keys: four groups of wavefronts that take tiles of all chunks in turn."""
+    test_query_gradient_in_workgroups_of_64_queries(heads, n, nk, P, dev)
+
+
 def test_backward_over_chunks_declines_what_it_does_not_cover(dev):
     q = torch.randn(1, 1, 128, 64, device=dev)
     k = [torch.randn(1, 1, 128, 64, device=dev)]
