@@ -32,7 +32,8 @@
 // A transposed copy of the tile beside it, fetched and written a second time, had these kernels at (copy : transpose reads, with the loads
 // above and two tiles a round; forward / dQ / dK and dV, us) 6 heads x 4050 x 4 chunks, head size 80 460 / 559 / 931 : 312 / 336 / 366; 24 x 1000 x 2, 128
 // 65 / 83 / 125 : 57 / 61 / 106; 24 x 739 x 5, 32 54 / 62 / 52 : 45 / 43 / 30; 8 x 4096 x 2, fp16 64 193 / 240 / 195 : 165 / 156 / 161. What is
-// left is one chain per wavefront, scores, exponentials, products, with two wavefronts a SIMD to fill its gaps.
+// left is one chain per wavefront, scores, exponentials, products, with two wavefronts a SIMD to fill its gaps, and, up to 64 columns where the
+// chip is full, a second block of rows in each (launch_fwd, launch_dq).
 //
 // Reference behaviour restated here:
 //   jigsaw/modules/attention/_functional/cores/math.py:69-78   (forward)
