@@ -86,10 +86,12 @@ __device__ __forceinline__ void parts8(const float* v, bf16x8_t (&part)[3]) {
 // are two or four times as many, and what their fewer rows leave free takes more tiles at once (four to eight groups a workgroup).
 // Forward / backward, us, before -> with it: 8 heads x 512 x 4 chunks at 128 47 / 84 -> 31 / 59, x 8 chunks at 32 39 / 59 -> 19 / 29. Forced, where 128 rows
 // have a workgroup for every second compute unit or more: 60 x 529 x 4, fp16 96 94 / 190 -> 125 / 209 (64 rows). At head size 32, whose workgroups
-// fit a compute unit several times, up to two of 64 rows each still gain: 28 x 931 x 7 84 / 156 -> 78 / 152.
+// fit a compute unit several times, up to two of 32 rows and three of 64 each still gain. Forward / backward of two launches, 64 : 32 rows: 44 x 322 x 8 28.3 / 54 : 21.0 / 47, 5 x 1734 x 6
+// 60.6 / 107 : 55.8 / 103, 30 x 531 x 3 19.0 / 38 : 14.8 / 34; beyond, 14 x 1782 x 3 48.9 / 108 : 57.1 / 117. 128 : 64 rows: 24 x 1388 x 7 158 / 284 : 127 / 252, 44 x 983 x 3 54.5 / 114 : 45.4 / 106,
+// 14 x 3095 x 7 340 / 678 : 269 / 605; beyond, 33 x 1497 x 5 128 / 262 : 127 / 262, 42 x 1968 x 8 337 / 828 : 375 / 822.
 inline int attn_width(long long rows, long long batch, int columns) {
-  if (cdiv(rows, 32) * batch <= cu_count()) return 1;
-  return cdiv(rows, 64) * batch <= (columns == 32 ? 2 : 1) * cu_count() ? 2 : 4;
+  if (cdiv(rows, 32) * batch <= (columns == 32 ? 2 : 1) * cu_count()) return 1;
+  return cdiv(rows, 64) * batch <= (columns == 32 ? 3 : 1) * cu_count() ? 2 : 4;
 }
 // (attn_wide.hip; dk, dv NULL: dQ and delta only)
 int attn_wide_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v, int nchunks,

@@ -916,7 +916,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void attn_wide_bwd_kernel(Chu
   else dkv_block<D, F16, 0, W, 4 / W, EXACT, true>(p, jg::block_at(blockIdx.x - dq_blocks, rest, k_rows, p.nchunks));
 }
 
-// Workgroups of 128 rows (attn_width: half of the CUs and more have one; at head size 32 all of them, twice): where some CU has none, two
+// Workgroups of 128 rows (attn_width: half of the CUs and more have one; at head size 32 all of them): where some CU has none, two
 // groups share the streamed side.
 bool two_groups(long long workgroups) { return workgroups < jg::cu_count(); }
 bool keys_from(const Args& a, long long n) { return (long long)a.sk * a.nchunks >= n; }
@@ -971,7 +971,8 @@ int launch_fwd(const ChunkTable& tab, const Args& a, long long batch, hipStream_
   };
   switch (jg::attn_width(a.sq, batch, D)) {
     case 1: return go(One{}, Most<D>{}, One{});
-    case 2: return go(Two{}, Four{}, One{});
+    case 2:  // (not past two a compute unit for keys that four groups cannot share: 600 x 64 x 1 at 32 8.9 us, 6.8 with 128 rows)
+      if (D > 32 || keys_from(a, 128) || jg::cdiv(a.sq, 64) * batch <= 2 * jg::cu_count()) return go(Two{}, Four{}, One{});
   }
   // 128 queries a workgroup, up to 64 columns: two blocks a wavefront in as many wavefronts, where the walk over the keys is long enough for the groups'
   // hand-over. One block : two, us, in four wavefronts: 48 x 1000 x 3 chunks, fp16 64 83 : 74, 28 x 1162 x 2, fp16 64 64 : 58, 16 x 2924 x 4 at 32

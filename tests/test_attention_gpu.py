@@ -694,7 +694,7 @@ def test_workgroups_of_every_width(h, sq, sk, P, d, dtype, dev):
 @pytest.mark.parametrize("h,sq,sk,d,P", [
     # workgroups of 128 rows on 256 compute units, up to 64 columns: two blocks of 32 rows a wavefront where the keys are many; blocks and
     # wavefronts without a row, key groups with fewer tiles, chunks shorter than 128 keys; four wavefronts, then eight
-    (520, 1, 129, 24, 16), (520, 33, 600, 32, 1), (300, 97, 161, 32, 13), (260, 65, 2049, 64, 1), (257, 128, 100, 64, 16), (260, 33, 257, 48, 4), (300, 31, 33, 40, 3),
+    (780, 1, 129, 24, 16), (780, 33, 600, 32, 1), (400, 97, 161, 32, 13), (520, 33, 600, 32, 1), (520, 33, 90, 32, 1), (260, 65, 2049, 64, 1), (257, 128, 100, 64, 16), (260, 33, 257, 48, 4), (300, 31, 33, 40, 3),
     (120, 130, 4100, 64, 1), (125, 129, 293, 56, 14),
 ])
 def test_workgroups_that_fill_the_chip(h, sq, sk, d, P, dtype, dev):
