@@ -1050,7 +1050,7 @@ int launch_dkv(const ChunkTable& tab, const Args& a, long long batch, hipStream_
 // Wider heads have one workgroup of the one launch on a compute unit: it is taken where all of them fit at once, priced in us by what a step took
 // there, by rows, with nine for a launch and what surrounds it. 13 x 102 x 2 at 128 21.8 : 12.7, 7 x 265 x 1 at 128 26.5 : 19.7, 2 x 2000 x 2 at 128
 // 119 : 93, 2 x 1000 x 3 at 96 52.3 : 33.0, 16 x 200 x 3 at 96 23.4 : 15.4, 40 x 90 x 4 at 80 27.4 : 19.2, 1 x 2500 x 2 at 96 92 : 66. Where it says no: 12 x 1180 x 1
-// at 96 53.8 : 74.6, 12 x 503 x 2 at 80 30.9 : 34.3, 8 x 512 x 4 at 128 56.8 : 61.5, 33 x 193 x 3 at 128 40.7 : 44.3 (but 30 x 140 x 4 at 128 40.8 : 34.7, more workgroups than fit).
+// at 96 53.8 : 74.6, 12 x 503 x 2 at 80 30.9 : 34.3, 11 x 845 x 2 at 80 48 : 53, 8 x 512 x 4 at 128 56.8 : 61.5, 33 x 193 x 3 at 128 40.7 : 44.3 (but 30 x 140 x 4 at 128 40.8 : 34.7, more workgroups than fit).
 double steps_alone(long long workgroups, long long steps, int wavefronts) {
   const long long each = jg::cdiv(workgroups, jg::cu_count());
   return (wavefronts == 8 ? (each == 1 ? 1.8 : 2.0 * each) : (each == 1 ? 1.1 : 1.0 * each)) * steps;
@@ -1078,7 +1078,7 @@ int one_launch_width(const Args& a, long long batch) {
   auto us_q = [](int w) { return w == 1 ? 1.2 : w == 2 ? 0.9 : 0.77; };
   auto us_k = [](int w) { return w == 1 ? 3.0 : w == 2 ? 2.05 : 1.75; };
   auto alone = [&](long long workgroups, double us, int wavefronts) { return us * (wavefronts == 8 ? 1.5 : 1.0) * jg::cdiv(workgroups, jg::cu_count()) + 9.0; };
-  double least = (D <= 96 ? 0.77 : 0.85) * (alone(blocks_q(q.w), us_q(q.w) * steps_q(q.ks), q.w * q.ks) + alone(blocks_k(k.w), us_k(k.w) * steps_k(k.ks), k.w * k.ks));
+  double least = (D <= 96 ? 0.72 : 0.85) * (alone(blocks_q(q.w), us_q(q.w) * steps_q(q.ks), q.w * q.ks) + alone(blocks_k(k.w), us_k(k.w) * steps_k(k.ks), k.w * k.ks));
   for (int w = 1; w <= 4; w *= 2) {
     const double one = std::max(us_q(w) * steps_q(4 / w), us_k(w) * steps_k(4 / w)) + 9.0;
     if (blocks_q(w) + blocks_k(w) <= jg::cu_count() && one < least) least = one, width = w;
