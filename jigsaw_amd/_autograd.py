@@ -4,12 +4,25 @@ from __future__ import annotations
 
 import torch
 from torch import _functorch
+from torch.autograd import forward_ad
 
 
 def native_nodes() -> bool:
-    """Whether a layer may leave its autograd node to the native host module: not under a functorch transform, in a trace or in
-    a compiled graph, which know the Python functions."""
-    return not (torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling())
+    """Whether a :class:`NativeFunction` may stand for a layer's own autograd function: not under a functorch transform or
+    forward-mode differentiation, in a trace or in a compiled graph, which know the layer's own."""
+    return not (torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0
+                or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling())
+
+
+def wants_grad(*tensors) -> bool:
+    """Whether autograd records what is computed from ``tensors`` (``None`` among them)."""
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+
+def saved_rows(ctx) -> tuple:
+    """``ctx.saved_tensors`` row-major, as the kernels' pointers take them: hooks of saved tensors (``saved_tensors_hooks``) may have
+    given them another layout."""
+    return tuple(t if t is None else t.contiguous() for t in ctx.saved_tensors)
 
 
 class PositionalFunction(torch.autograd.Function):
@@ -24,3 +37,24 @@ class PositionalFunction(torch.autograd.Function):
         if kwargs or torch._C._are_functorch_transforms_active():
             return super().apply(*args, **kwargs)
         return super(torch.autograd.Function, cls).apply(*_functorch.utils.unwrap_dead_wrappers(args))
+
+
+class NativeFunction(torch.autograd.Function):
+    """The node behind a result that the native host module has computed already: ``apply(result, saved, rest, *inputs)``
+    hands ``result`` out with ``backward(ctx, grad)`` of the subclass behind it, which finds the tensors ``saved`` in
+    ``ctx.saved_tensors`` and ``rest`` as it was given, and returns ``(None, None, None, *gradients of inputs)``.
+
+    What it saves on a layer's own function is that function's ``forward`` and ``setup_context``: of steps that wait for the host 10 us
+    in 121 (convolution), 8 in 104 (GroupNorm) and 5 in 118 (sharded LayerNorm). The node is a Python function's all the same, so that
+    the collector sees what it keeps (an exchange that keeps the result makes a cycle through it) and compiled autograd can
+    record it; a node in C++ takes 15 to 20 us less and can do neither. Projections and Swin block gain nothing from it."""
+
+    @classmethod
+    def apply(cls, result, saved, rest, *inputs):
+        return super(torch.autograd.Function, cls).apply((result,), saved, rest, *inputs)
+
+    @staticmethod
+    def forward(ctx, result, saved, rest, *inputs):  # noqa: D102
+        ctx.save_for_backward(*saved)
+        ctx.rest = rest
+        return result[0]

@@ -29,7 +29,7 @@ from typing import Any, Protocol
 import torch
 
 from . import _lib
-from ._autograd import PositionalFunction, native_nodes
+from ._autograd import NativeFunction, PositionalFunction, native_nodes, wants_grad
 from .halo import (HaloGeometry, halo_assemble, halo_fold, halo_fold_border_, halo_gather_axis, halo_pack,
                    halo_scatter_add_axis, new_strips, spans_fit_the_strips, strip_table)
 
@@ -1072,6 +1072,27 @@ def conv_halo_nway(x, w, b, stride, padding, dilation, spatial_groups, channel_g
     return y, x_aug
 
 
+def _backward_by_plan(step, g, x_aug, weight, stride, padding, dilation, local_in_spatial, spatial_groups, config, need):
+    """``(g_x, g_w, g_b)`` of a layer that the native plan ``step`` runs, or ``None`` where it does not take these tensors."""
+    need_x, need_w, need_b = need
+    stream = _lib.stream_handle(g.device)
+    parts = step.backward(g, x_aug, weight, need_x, need_w, need_w and need_b, stream)
+    if parts is None:
+        return None
+    part, g_w, g_b, send, folded, left = parts
+    if need_b and g_b is None:
+        g_b = config.grad_bias(g.contiguous())
+    if not need_x:
+        return None, g_w, g_b
+    recv = config.halo_exchange.backward(send) if step.sends else {}
+    g_x = step.finish(part, folded, recv, stream, left)
+    if g_x is None:  # strips in another layout
+        ranks, sizes = _mesh_position(spatial_groups)
+        geom = HaloGeometry.for_conv(local_in_spatial, weight.shape[-config.n_spatial :], stride, padding, dilation, ranks, sizes)
+        g_x = halo_fold_border_(part, recv, geom) if folded else halo_fold(part, recv, geom)
+    return g_x, g_w, g_b
+
+
 def conv_halo_nway_backward(
     grad_output, x_aug, weight, stride, padding, dilation, local_in_spatial, spatial_groups, channel_group, config,
     need=(True, True), x_tile=None,
@@ -1093,19 +1114,11 @@ def conv_halo_nway_backward(
     g_w = g_b = None
     if x_tile is None and g.is_cuda and x_aug.dtype == g.dtype and not getattr(x_aug, "_jg_frame_only", False):
         step = _step_for(config, (*x_aug.shape[:2], *local_in_spatial), x_aug, weight, stride, padding, dilation, ranks, sizes)
-        stream = _lib.stream_handle(g.device) if step is not None else 0
-        parts = step.backward(g, x_aug, weight, need_x, need_w, need_w and need_b, stream) if step is not None else None
-        if parts is not None:
-            part, g_w, g_b, send, folded, left = parts
-            if need_b and g_b is None:
-                g_b = config.grad_bias(g.contiguous())
-            if not need_x:
-                return done(None)
-            recv = config.halo_exchange.backward(send) if step.sends else {}
-            g_x = step.finish(part, folded, recv, stream, left)
-            if g_x is None:
-                geom = HaloGeometry.for_conv(local_in_spatial, weight.shape[-n:], stride, padding, dilation, ranks, sizes)
-                g_x = halo_fold_border_(part, recv, geom) if folded else halo_fold(part, recv, geom)
+        got = None
+        if step is not None:
+            got = _backward_by_plan(step, g, x_aug, weight, stride, padding, dilation, local_in_spatial, spatial_groups, config, (need_x, need_w, need_b))
+        if got is not None:
+            g_x, g_w, g_b = got
             return done(g_x)
     local_padding = _local_padding(padding, sizes)
     kwargs = {"stride": stride, "padding": local_padding, "dilation": dilation, "groups": int(getattr(config, "groups_local", 1))}
@@ -1305,25 +1318,34 @@ class _Received:
         return getattr(self._exchange, name)
 
 
-def _backward_without_plan(g, x_aug, weight, need_x, need_w, need_b, local_in_spatial, stride, padding, dilation, spatial_groups, channel_group, config):
-    """The backward of a layer whose native node declined what it got (saved tensors that came back in another layout)."""
-    if x_aug.dtype != weight.dtype:
-        x_aug = x_aug.to(weight.dtype)
-    return conv_halo_nway_backward(g, x_aug, weight, stride, padding, dilation, local_in_spatial, spatial_groups, channel_group, config,
-                                   need=(need_x, need_w, need_b))
+class _NativeConvNd(NativeFunction):
+    """``_ConvNd`` of a layer that the native plan runs as it is: the same launches, less of the host. ``rest`` is the
+    plan, ``_ConvNd``'s arguments from ``stride`` on and the extents of the tile."""
 
+    @staticmethod
+    def forward(ctx, *args):  # noqa: D102
+        ctx.set_materialize_grads(False)
+        return NativeFunction.forward(ctx, *args)
 
-def _fold_without_plan(part, folded, recv, weight, local_in_spatial, stride, padding, dilation, spatial_groups, channel_group, config):
-    """The last step of the backward where the neighbours' strips are not what the plan takes."""
-    ranks, sizes = _mesh_position(spatial_groups)
-    geom = HaloGeometry.for_conv(local_in_spatial, weight.shape[-config.n_spatial:], stride, padding, dilation, ranks, sizes)
-    return halo_fold_border_(part, recv, geom) if folded else halo_fold(part, recv, geom)
+    @staticmethod
+    def backward(ctx, g):  # noqa: D102
+        if g is None:
+            return (None,) * 6
+        x_aug, weight = ctx.saved_tensors
+        step, (stride, padding, dilation, spatial_groups, channel_group, config), local = ctx.rest
+        need = ctx.needs_input_grad[3:]
+        got = _backward_by_plan(step, g, x_aug, weight, stride, padding, dilation, local, spatial_groups, config, need)
+        if got is None:  # hooks of the saved tensors have given them another layout or type
+            if x_aug.dtype != weight.dtype:
+                x_aug = x_aug.to(weight.dtype)
+            got = conv_halo_nway_backward(g, x_aug, weight, stride, padding, dilation, local, spatial_groups, channel_group, config, need=need)
+        return None, None, None, *got
 
 
 class _ConvNd(PositionalFunction):
     """Autograd function of the distributed convolution
     (jigsaw/modules/convolution/_conv/functional.py:28-169), HIP kernels inside. Layers that the native plan runs as they
-    are get a node of the native host module instead (``host.conv_apply``): the same launches, less of the host."""
+    are get the node of :class:`_NativeConvNd` instead."""
 
     @classmethod
     def apply(cls, *args, **kwargs):
@@ -1336,18 +1358,21 @@ class _ConvNd(PositionalFunction):
             return super().apply(*args)
         step = _step_for(config, x.shape, x, w, stride, padding, dilation, *_mesh_position(spatial_groups))
         host = _lib.host()
-        if step is None or type(step) is not host.Step or not host.conv_takes(step, x, w, b):
+        if step is None or type(step) is not host.Step or not step.takes(x, w, b):
             return super().apply(*args)
         stream = _lib.stream_handle(x.device)
         exchange = config.halo_exchange
         with torch.no_grad():
             recv = exchange.forward(step.pack(x, stream)) if step.sends else {}
-        done = host.conv_apply(step, x, recv, w, b, args[3:], stream)
+        done = step.forward(x, recv, w, b, stream)
         if done is None:  # strips in another layout
             config = copy.copy(config)
             config.halo_exchange = _Received(exchange, recv)
             return super().apply(*args[:8], config)
-        return done
+        if not wants_grad(x, w, b):
+            return done
+        y, x_aug = done
+        return _NativeConvNd.apply(y, (x_aug, w), (step, args[3:], x.shape[2:]), x, w, b), x_aug
 
     @staticmethod
     def forward(x, weight, bias, stride, padding, dilation, spatial_groups, channel_group, config):  # noqa: D102

@@ -13,11 +13,6 @@
 //
 // What a Step does not take (a strip of another shape or layout, tensors of mixed types) it declines by returning
 // None before anything is launched; the callers' Python route then names the error or handles the case.
-#include <c10/hip/HIPStream.h>
-#include <torch/csrc/autograd/VariableTypeUtils.h>
-#include <torch/csrc/autograd/functions/utils.h>
-#include <torch/csrc/autograd/python_cpp_function.h>
-#include <torch/csrc/autograd/saved_variable.h>
 #include <torch/extension.h>
 
 #include <algorithm>
@@ -43,9 +38,7 @@ struct Strip {
 };
 
 void check(int rc, const char* what) {
-  if (rc == JG_OK) return;
-  const py::gil_scoped_acquire gil;
-  py::module_::import("jigsaw_amd._lib").attr("check")(rc, what);
+  if (rc != JG_OK) py::module_::import("jigsaw_amd._lib").attr("check")(rc, what);
 }
 
 Shape to_shape(const py::handle& seq) {
@@ -112,29 +105,16 @@ class Step {
   // padded one, or with `folded` the own tile's, to which only the neighbours' blocks are still missing. The
   // bias gradient is None where only the separate kernels cover the layer. Sums left (None, or for `finish`): what the weight
   // and bias gradient still miss.
-  py::object backward(const at::Tensor& g, const at::Tensor& x_aug, const at::Tensor& w, bool need_x, bool need_w, bool need_b, uintptr_t stream) {
-    Parts p;
-    if (!backward_parts(g, x_aug, w, need_x, need_w, need_b, stream, p)) return py::none();
-    auto given = [](const at::Tensor& t) -> py::object { return t.defined() ? py::cast(t) : py::none(); };
-    return py::make_tuple(given(p.gx), given(p.gw), given(p.gb), p.send, p.folded, p.left.sums.kind != 0 ? py::cast(std::move(p.left)) : py::none());
-  }
-
-  struct Parts {
-    at::Tensor gx, gw, gb;
-    py::dict send;
-    bool folded = false;
-    SumsLeft left;
-  };
-
-  // `backward` as tensors; false: declined, nothing launched
-  bool backward_parts(const at::Tensor& g_any, const at::Tensor& x_aug, const at::Tensor& w_any, bool need_x, bool need_w, bool need_b,
-                      uintptr_t stream, Parts& p) {
+  py::object backward(const at::Tensor& g_any, const at::Tensor& x_aug, const at::Tensor& w_any, bool need_x, bool need_w, bool need_b,
+                      uintptr_t stream) {
     if (g_any.sizes() != at::IntArrayRef(y_shape_) || x_aug.sizes() != at::IntArrayRef(padded_) || !x_aug.is_contiguous() ||
         w_any.sizes() != at::IntArrayRef(w_shape_) || !same_kind(g_any, x_aug) || !same_kind(w_any, x_aug))
-      return false;
+      return py::none();
     at::AutoDispatchBelowADInplaceOrView below;
     void* const s = reinterpret_cast<void*>(stream);
     const at::Tensor g = g_any.contiguous(), w = w_any.contiguous();
+    py::object gw = py::none(), gb = py::none(), gx = py::none(), send = py::dict(), left = py::none();
+    bool folded = false;
     SumsLeft later;
     if (need_w) {
       const at::Tensor gw_t = at::empty(w_shape_, g.options());
@@ -152,13 +132,13 @@ class Step {
         }
         if (rc != JG_ERR_UNSUPPORTED) {
           check(rc, "jg_conv_wgrad_bias");
-          p.gb = gb_t;
+          gb = py::cast(gb_t);
         }
       }
       if (rc == JG_ERR_UNSUPPORTED)
         check(jg_conv_wgrad(gw_t.data_ptr(), x_aug.data_ptr(), g.data_ptr(), &desc_, code_, address(ws), nbytes_[JG_CONV_WGRAD], s),
               "jg_conv_wgrad");
-      p.gw = gw_t;
+      gw = py::cast(gw_t);
     }
     if (need_x) {
       const at::Tensor ws = scratch(nbytes_[JG_CONV_DGRAD], g);
@@ -171,43 +151,40 @@ class Step {
                                           nbytes_[JG_CONV_DGRAD], s);
         if (rc != JG_ERR_UNSUPPORTED) {
           check(rc, "jg_conv_dgrad_fold");
-          p.gx = own;
-          p.send = out;
-          p.folded = true;
+          gx = py::cast(own);
+          send = out;
+          folded = true;
         } else {
           fold_.store(false, std::memory_order_relaxed);
         }
       }
       if (later.sums.kind != 0) {
-        if (p.folded) {
-          p.left = std::move(later);
+        if (folded) {
+          left = py::cast(std::move(later));
         } else {
           check(jg_conv_reduce(&later.sums, s), "jg_conv_reduce");
           later.held.clear();
         }
       }
-      if (!p.folded) {
+      if (!folded) {
         const at::Tensor need = at::empty(padded_, g.options());
         check(jg_conv_dgrad(need.data_ptr(), w.data_ptr(), g.data_ptr(), &desc_, code_, address(ws), nbytes_[JG_CONV_DGRAD], s),
               "jg_conv_dgrad");
-        p.gx = need;
-        if (!send_bwd_.empty()) p.send = cut(need, send_bwd_, own_, 1, stream);
+        gx = py::cast(need);
+        if (!send_bwd_.empty()) send = cut(need, send_bwd_, own_, 1, stream);
       }
     }
-    return true;
+    return py::make_tuple(gx, gw, gb, send, folded, left);
   }
 
   // The own tile's gradient from what `backward` returned and the neighbours' blocks, or None. The sums left are done in any case.
   py::object finish(const at::Tensor& part, bool folded, const py::object& recv, uintptr_t stream, const py::object& left) const {
-    const at::Tensor gx = finished(part, folded, recv, stream, left.is_none() ? nullptr : &left.cast<const SumsLeft&>().sums);
-    return gx.defined() ? py::cast(gx) : py::none();
-  }
-  at::Tensor finished(const at::Tensor& part, bool folded, const py::object& recv, uintptr_t stream, const jg_conv_reduction* sums) const {
     const void* tab[27] = {};
     void* const s = reinterpret_cast<void*>(stream);
+    const jg_conv_reduction* const sums = left.is_none() ? nullptr : &left.cast<const SumsLeft&>().sums;
     if (!table(recv, recv_bwd_, part, tab)) {
       if (sums != nullptr) check(jg_conv_reduce(sums, s), "jg_conv_reduce");
-      return at::Tensor();
+      return py::none();
     }
     at::AutoDispatchBelowADInplaceOrView below;
     at::Tensor gx = part;
@@ -221,18 +198,13 @@ class Step {
       check(jg_halo_fold_border_reduce_3d(gx.data_ptr(), tab, &theirs_, code_, sums, s), "jg_halo_fold_border_reduce_3d");
     else if (folded || !same_)
       check(jg_halo_fold_border_3d(gx.data_ptr(), tab, &theirs_, code_, s), "jg_halo_fold_border_3d");
-    return gx;
+    return py::cast(gx);
   }
 
   // Whether `forward` takes these, whatever strips arrive
   bool takes(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& b) const {
-    return x.sizes() == at::IntArrayRef(x_shape_) && x.is_contiguous() && w.sizes() == at::IntArrayRef(w_shape_) && same_kind(w, x) &&
+    return x.has_storage() && x.sizes() == at::IntArrayRef(x_shape_) && x.is_contiguous() && w.sizes() == at::IntArrayRef(w_shape_) && same_kind(w, x) &&
            (!b || (same_kind(*b, x) && b->dim() == 1 && b->size(0) == w_shape_[0]));
-  }
-  py::tuple local_size() const {
-    py::tuple t(x_shape_.size() - 2);
-    for (size_t a = 2; a < x_shape_.size(); ++a) t[a - 2] = py::int_(x_shape_[a]);
-    return t;
   }
 
  private:
@@ -326,7 +298,7 @@ int code_of(const at::Tensor& t) {
     default: return -1;
   }
 }
-bool on_gpu(const at::Tensor& t) { return t.is_cuda() && t.is_contiguous(); }
+bool on_gpu(const at::Tensor& t) { return t.is_cuda() && t.is_contiguous() && t.has_storage(); }
 bool aligned(const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
 void* pointer(uintptr_t p) { return reinterpret_cast<void*>(p); }
 
@@ -427,49 +399,45 @@ void ln_recentre(const at::Tensor& var, const at::Tensor& own, const at::Tensor&
 }
 
 // (y, x_norm, var + eps) in w's type; `std` gets the root. x, w and b as the Python route has them at this point.
-void ln_normalise(const at::Tensor& x, const at::Tensor& mean, const at::Tensor& var, const at::Tensor& std, const at::Tensor& w,
-                  const c10::optional<at::Tensor>& b, double eps, uintptr_t stream, at::Tensor& y, at::Tensor& x_norm, at::Tensor& var_eps) {
+py::tuple ln_apply(const at::Tensor& x, const at::Tensor& mean, const at::Tensor& var, const at::Tensor& std, const at::Tensor& w,
+                   const c10::optional<at::Tensor>& b, double eps, uintptr_t stream) {
   at::AutoDispatchBelowADInplaceOrView below;
   const int64_t cols = x.size(-1), rows = x.numel() / cols;
-  y = at::empty(x.sizes(), w.options()), x_norm = at::empty(x.sizes(), w.options()), var_eps = at::empty(mean.sizes(), w.options());
+  const at::Tensor y = at::empty(x.sizes(), w.options()), x_norm = at::empty(x.sizes(), w.options()), var_eps = at::empty(mean.sizes(), w.options());
   check(jg_ln_apply2(y.data_ptr(), x_norm.data_ptr(), std.data_ptr<float>(), var_eps.data_ptr(), x.data_ptr(), mean.data_ptr<float>(),
                      var.data_ptr<float>(), w.data_ptr(), b ? b->data_ptr() : nullptr, rows, cols, (float)eps, code_of(x), code_of(w), pointer(stream)),
         "jg_ln_apply2");
-}
-py::tuple ln_apply(const at::Tensor& x, const at::Tensor& mean, const at::Tensor& var, const at::Tensor& std, const at::Tensor& w,
-                   const c10::optional<at::Tensor>& b, double eps, uintptr_t stream) {
-  at::Tensor y, x_norm, var_eps;
-  ln_normalise(x, mean, var, std, w, b, eps, stream, y, x_norm, var_eps);
   return py::make_tuple(y, x_norm, var_eps);
 }
 
-// (mean of g w, sum of g w x_norm, gw, gb): the backward before the collectives; parameter gradients in `grad_type`
-bool ln_sums(const at::Tensor& g, const at::Tensor& x_norm, const at::Tensor& w, const at::Tensor& std, bool need_w, bool need_b,
-             const at::ScalarType grad_type, uintptr_t stream, at::Tensor& mean, at::Tensor& dot, at::Tensor& gw, at::Tensor& gb) {
+// Whether ln_apply takes these as they are: parameters in the type that y gets, nothing to be copied
+bool ln_takes(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& b, const at::ScalarType type) {
+  auto parameter = [&](const at::Tensor& t) {
+    return on_gpu(t) && t.scalar_type() == type && t.device() == x.device() && t.dim() == 1 && t.size(0) == x.size(-1);
+  };
+  return x.dim() >= 1 && x.numel() > 0 && on_gpu(x) && code_of(x) >= 0 && parameter(w) && code_of(w) >= 0 && (!b || parameter(*b));
+}
+
+// (mean of g w, sum of g w x_norm, gw, gb): the backward before the collectives; parameter gradients in `like`'s type
+py::object ln_partial_bwd(const at::Tensor& g, const at::Tensor& x_norm, const at::Tensor& w, const at::Tensor& std, bool need_w, bool need_b,
+                          const at::ScalarType grad_type, uintptr_t stream) {
   if (g.numel() == 0 || !on_gpu(g) || !on_gpu(x_norm) || !on_gpu(w) || g.scalar_type() != x_norm.scalar_type() || g.sizes() != x_norm.sizes() ||
       w.scalar_type() != g.scalar_type() || code_of(g) < 0)
-    return false;
+    return py::none();
   at::AutoDispatchBelowADInplaceOrView below;
   const int64_t cols = g.size(-1), rows = g.numel() / cols;
   Shape shape{2};
   shape.append(std.sizes().begin(), std.sizes().end());
   const List t = at::empty(shape, std.options()).unbind(0);
   const auto options = g.options().dtype(grad_type);
-  mean = t[0], dot = t[1];
-  gw = need_w ? at::empty({cols}, options) : at::Tensor(), gb = need_b ? at::empty({cols}, options) : at::Tensor();
+  const at::Tensor gw = need_w ? at::empty({cols}, options) : at::Tensor(), gb = need_b ? at::empty({cols}, options) : at::Tensor();
   const size_t nbytes = need_w || need_b ? jg_ln_bwd_workspace_bytes(rows, cols) : 0;
   const at::Tensor ws = at::empty({(int64_t)(nbytes > 4 ? nbytes : 4)}, g.options().dtype(at::kByte));
   const int code = grad_type == at::kFloat ? JG_F32 : grad_type == at::kBFloat16 ? JG_BF16 : JG_F16;
   check(jg_ln_partial_bwd2(t[0].data_ptr<float>(), t[1].data_ptr<float>(), need_w ? gw.data_ptr() : nullptr, need_b ? gb.data_ptr() : nullptr, code,
                            g.data_ptr(), x_norm.data_ptr(), w.data_ptr(), rows, cols, code_of(g), ws.data_ptr(), nbytes, pointer(stream)),
         "jg_ln_partial_bwd2");
-  return true;
-}
-py::object ln_partial_bwd(const at::Tensor& g, const at::Tensor& x_norm, const at::Tensor& w, const at::Tensor& std, bool need_w, bool need_b,
-                          const at::ScalarType grad_type, uintptr_t stream) {
-  at::Tensor mean, dot, gw, gb;
-  if (!ln_sums(g, x_norm, w, std, need_w, need_b, grad_type, stream, mean, dot, gw, gb)) return py::none();
-  return py::make_tuple(mean, dot, need_w ? py::cast(gw) : py::none(), need_b ? py::cast(gb) : py::none());
+  return py::make_tuple(t[0], t[1], need_w ? py::cast(gw) : py::none(), need_b ? py::cast(gb) : py::none());
 }
 
 at::Tensor ln_bwd_apply(const at::Tensor& g, const at::Tensor& x_norm, const at::Tensor& w, const at::Tensor& mean, const at::Tensor& dot,
@@ -488,42 +456,33 @@ bool like_channels(const c10::optional<at::Tensor>& t, const at::Tensor& x) {
 }
 
 // (y, the copy of x or None, mean, rstd)
-bool gn_output(const at::Tensor& x, int64_t groups, const c10::optional<at::Tensor>& w, const c10::optional<at::Tensor>& b, double eps, bool keep,
-               uintptr_t stream, at::Tensor& y, at::Tensor& kept, at::Tensor& mean, at::Tensor& rstd) {
-  if (x.dim() < 2 || x.numel() == 0 || !on_gpu(x) || code_of(x) < 0 || !like_channels(w, x) || !like_channels(b, x)) return false;
+py::object gn_forward(const at::Tensor& x, int64_t groups, const c10::optional<at::Tensor>& w, const c10::optional<at::Tensor>& b, double eps,
+                      bool keep, uintptr_t stream) {
+  if (x.dim() < 2 || x.numel() == 0 || !on_gpu(x) || code_of(x) < 0 || !like_channels(w, x) || !like_channels(b, x)) return py::none();
   at::AutoDispatchBelowADInplaceOrView below;
   const int64_t n = x.size(0), c = x.size(1), s = x.numel() / (n * c);
-  y = at::empty_like(x), kept = keep ? at::empty_like(x) : at::Tensor();
+  const at::Tensor y = at::empty_like(x), kept = keep ? at::empty_like(x) : at::Tensor();
   const List t = at::empty({2, n, groups}, x.options().dtype(at::kFloat)).unbind(0);
-  mean = t[0], rstd = t[1];
   const size_t nbytes = jg_gn_workspace_bytes(n, c, s);
   const at::Tensor ws = at::empty({(int64_t)nbytes}, x.options().dtype(at::kByte));
   check(jg_gn_forward_keep(y.data_ptr(), keep ? kept.data_ptr() : nullptr, t[0].data_ptr<float>(), t[1].data_ptr<float>(), x.data_ptr(),
                            w ? w->data_ptr() : nullptr, b ? b->data_ptr() : nullptr, n, c, s, groups, (float)eps, code_of(x), ws.data_ptr(), nbytes,
                            pointer(stream)),
         "jg_gn_forward_keep");
-  return true;
-}
-py::object gn_forward(const at::Tensor& x, int64_t groups, const c10::optional<at::Tensor>& w, const c10::optional<at::Tensor>& b, double eps,
-                      bool keep, uintptr_t stream) {
-  at::Tensor y, kept, mean, rstd;
-  if (!gn_output(x, groups, w, b, eps, keep, stream, y, kept, mean, rstd)) return py::none();
-  return py::make_tuple(y, keep ? py::cast(kept) : py::none(), mean, rstd);
+  return py::make_tuple(y, keep ? py::cast(kept) : py::none(), t[0], t[1]);
 }
 
 // (gx, gw, gb); the parameter gradients in `grad_type`
-bool gn_gradients(const at::Tensor& g, const at::Tensor& x, const at::Tensor& mean, const at::Tensor& rstd, const c10::optional<at::Tensor>& w,
-                  int64_t groups, bool need_x, bool need_w, bool need_b, const at::ScalarType grad_type, uintptr_t stream, at::Tensor& gx,
-                  at::Tensor& gw, at::Tensor& gb) {
+py::object gn_backward(const at::Tensor& g, const at::Tensor& x, const at::Tensor& mean, const at::Tensor& rstd, const c10::optional<at::Tensor>& w,
+                       int64_t groups, bool need_x, bool need_w, bool need_b, const at::ScalarType grad_type, uintptr_t stream) {
   if (g.numel() == 0 || !on_gpu(g) || !on_gpu(x) || g.scalar_type() != x.scalar_type() || g.sizes() != x.sizes() || code_of(g) < 0 ||
       !like_channels(w, x))
-    return false;
+    return py::none();
   at::AutoDispatchBelowADInplaceOrView below;
   const int64_t n = x.size(0), c = x.size(1), s = x.numel() / (n * c);
   const auto options = g.options().dtype(grad_type);
-  gx = need_x ? at::empty_like(g) : at::Tensor();
-  gw = need_w ? at::empty({c}, options) : at::Tensor();
-  gb = need_b ? at::empty({c}, options) : at::Tensor();
+  const at::Tensor gx = need_x ? at::empty_like(g) : at::Tensor(), gw = need_w ? at::empty({c}, options) : at::Tensor(),
+                   gb = need_b ? at::empty({c}, options) : at::Tensor();
   const size_t nbytes = jg_gn_workspace_bytes(n, c, s);
   const at::Tensor ws = at::empty({(int64_t)nbytes}, x.options().dtype(at::kByte));
   const int code = grad_type == at::kFloat ? JG_F32 : grad_type == at::kBFloat16 ? JG_BF16 : JG_F16;
@@ -531,263 +490,8 @@ bool gn_gradients(const at::Tensor& g, const at::Tensor& x, const at::Tensor& me
                        mean.data_ptr<float>(), rstd.data_ptr<float>(), w ? w->data_ptr() : nullptr, n, c, s, groups, code_of(x), code,
                        ws.data_ptr(), nbytes, pointer(stream)),
         "jg_gn_backward");
-  return true;
-}
-py::object gn_backward(const at::Tensor& g, const at::Tensor& x, const at::Tensor& mean, const at::Tensor& rstd, const c10::optional<at::Tensor>& w,
-                       int64_t groups, bool need_x, bool need_w, bool need_b, const at::ScalarType grad_type, uintptr_t stream) {
-  at::Tensor gx, gw, gb;
-  if (!gn_gradients(g, x, mean, rstd, w, groups, need_x, need_w, need_b, grad_type, stream, gx, gw, gb)) return py::none();
   auto given = [](const at::Tensor& t) -> py::object { return t.defined() ? py::cast(t) : py::none(); };
   return py::make_tuple(given(gx), given(gw), given(gb));
-}
-
-// ---- autograd nodes of the convolution, the sharded LayerNorm's and GroupNorm's `y` (conv._ConvNd, layernorm.layer_norm,
-// groupnorm.group_norm) and, below, the projections and the Swin block: their backward is called by the engine without a Python function in between. The engine runs it on
-// a thread of its own, and that thread's Python (the frame, the context, a tuple of saved tensors, the functions in between) cost up to
-// 35 us of a step that takes 100 to 140 in all. What only Python can do (functorch transforms, forward-mode tangents, tracing, casts, copies)
-// stays on the classes in conv.py, layernorm.py and groupnorm.py: their callers ask for it (_autograd.native_nodes) or
-// get None back from here, before anything is launched.
-using torch::autograd::Node;
-using torch::autograd::SavedVariable;
-using torch::autograd::variable_list;
-
-// A Python object in a node, which goes on whatever thread drops the node last
-class Held {
- public:
-  Held() = default;
-  Held(const Held&) = delete;
-  Held& operator=(const Held&) = delete;
-  ~Held() {
-    if (p_ == nullptr || !Py_IsInitialized()) return;
-    const py::gil_scoped_acquire gil;
-    Py_DECREF(p_);
-  }
-  void hold(py::object o) { p_ = o.release().ptr(); }  // once
-  py::handle get() const { return p_; }
-
- private:
-  PyObject* p_ = nullptr;
-};
-
-// What a Python callback raised, as the engine hands it to whoever called it
-[[noreturn]] void raise_as_is(py::error_already_set& e) {
-  e.restore();
-  python_error err;
-  err.persist();
-  throw std::move(err);
-}
-
-uintptr_t current_stream(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(c10::hip::getCurrentHIPStream(t.device().index()).stream()); }
-
-bool has_tangent(const at::Tensor& t) { return torch::autograd::isFwGradDefined(t); }
-bool has_tangent(const c10::optional<at::Tensor>& t) { return torch::autograd::isFwGradDefined(t); }
-template <typename W, typename B>
-bool any_tangent(const at::Tensor& x, const W& w, const B& b) { return has_tangent(x) || has_tangent(w) || has_tangent(b); }
-at::Tensor given(const c10::optional<at::Tensor>& t) { return t ? *t : at::Tensor(); }
-
-// A node behind y, fed by x, w and b
-template <typename N>
-std::shared_ptr<N> node_of(const at::Tensor& x, const at::Tensor& w, const at::Tensor& b) {
-  std::shared_ptr<N> node(new N(), torch::autograd::deleteNode);
-  node->set_next_edges(torch::autograd::collect_next_edges(x, w, b));
-  return node;
-}
-
-// The gradient of an output nobody used: zeros where the Python function gets zeros
-at::Tensor defined_or_zeros(const Node& node, const at::Tensor& g) { return g.defined() ? g : node.input_metadata(0).zeros_like(); }
-
-struct ConvNode : Node {
-  std::string name() const override { return "_ConvNdBackward"; }
-  void release_variables() override {
-    const std::lock_guard<std::mutex> lock(mutex_);
-    x_aug.reset_data();
-    w.reset_data();
-  }
-  variable_list apply(variable_list&& grads) override {
-    variable_list out(3);
-    const at::Tensor g = grads[0];
-    if (!g.defined()) return out;
-    at::Tensor padded, weight;
-    {
-      const std::lock_guard<std::mutex> lock(mutex_);
-      padded = x_aug.unpack();
-      weight = w.unpack();
-    }
-    const bool need_x = should_compute_output(0), need_w = should_compute_output(1), need_b = should_compute_output(2);
-    const uintptr_t stream = current_stream(g);
-    const py::gil_scoped_acquire gil;
-    try {
-      const py::tuple rest = py::reinterpret_borrow<py::tuple>(args.get());  // stride, padding, dilation, spatial groups, channel group, config
-      const py::handle config = rest[5];
-      Step& plan = step.get().cast<Step&>();
-      Step::Parts p;
-      if (!plan.backward_parts(g, padded, weight, need_x, need_w, need_w && need_b, stream, p)) {
-        const py::tuple all = py::module_::import("jigsaw_amd.conv").attr("_backward_without_plan")(g, padded, weight, need_x, need_w, need_b, plan.local_size(), *rest);
-        for (size_t i = 0; i < 3; ++i)
-          if (!all[i].is_none()) out[i] = all[i].cast<at::Tensor>();
-        return out;
-      }
-      if (need_b && !p.gb.defined()) p.gb = config.attr("grad_bias")(g.contiguous()).cast<at::Tensor>();
-      out[1] = p.gw;
-      out[2] = p.gb;
-      if (!need_x) return out;
-      const py::object recv = plan.sends() ? py::object(config.attr("halo_exchange").attr("backward")(p.send)) : py::dict();
-      out[0] = plan.finished(p.gx, p.folded, recv, stream, p.left.sums.kind != 0 ? &p.left.sums : nullptr);
-      if (!out[0].defined())
-        out[0] = py::module_::import("jigsaw_amd.conv").attr("_fold_without_plan")(p.gx, p.folded, recv, weight, plan.local_size(), *rest).cast<at::Tensor>();
-    } catch (py::error_already_set& e) {
-      raise_as_is(e);
-    }
-    return out;
-  }
-
-  Held step, args;
-  SavedVariable x_aug, w;
-};
-
-// (y, x_aug) with the node behind y where a gradient is wanted, or None where the strips are not what the plan takes
-py::object conv_apply(const py::object& step, const at::Tensor& x, const py::object& recv, const at::Tensor& w, const c10::optional<at::Tensor>& b,
-                      const py::tuple& args, uintptr_t stream) {
-  const py::object done = step.cast<Step&>().forward(x, recv, w, b, stream);
-  if (done.is_none() || !torch::autograd::compute_requires_grad(x, w, given(b))) return done;
-  const py::tuple both = done;
-  const auto node = node_of<ConvNode>(x, w, given(b));
-  node->step.hold(step);
-  node->args.hold(args);
-  node->x_aug = SavedVariable(both[1].cast<at::Tensor>(), false);
-  node->w = SavedVariable(w, false);
-  const at::Tensor y = both[0].cast<at::Tensor>();
-  torch::autograd::set_history(y, node);
-  return done;
-}
-// Whether conv_apply may run: everything but the strips is as the plan has it, and there are no tangents
-bool conv_takes(const Step& step, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& b) {
-  return step.takes(x, w, b) && !any_tangent(x, w, b);
-}
-
-struct GroupNormNode : Node {
-  std::string name() const override { return "_GroupNormOutputBackward"; }
-  void release_variables() override {
-    const std::lock_guard<std::mutex> lock(mutex_);
-    for (SavedVariable* v : {&x, &mean, &rstd, &w}) v->reset_data();
-  }
-  variable_list apply(variable_list&& grads) override {
-    variable_list out(3);
-    const at::Tensor g = defined_or_zeros(*this, grads[0]);
-    at::Tensor x_, mean_, rstd_;
-    c10::optional<at::Tensor> w_;
-    {
-      const std::lock_guard<std::mutex> lock(mutex_);
-      x_ = x.unpack();
-      mean_ = mean.unpack();
-      rstd_ = rstd.unpack();
-      if (has_w) w_ = w.unpack();
-    }
-    // hooks of the saved tensors may have given them another layout
-    x_ = x_.contiguous();
-    if (w_) w_ = w_->contiguous();
-    const bool done = gn_gradients(g.contiguous(), x_, mean_.contiguous(), rstd_.contiguous(), w_, groups, should_compute_output(0),
-                                   should_compute_output(1), should_compute_output(2), has_w || has_b ? x_.scalar_type() : at::kFloat,
-                                   current_stream(x_), out[0], out[1], out[2]);
-    TORCH_CHECK(done, "group_norm: what the backward got is not what the forward saved");
-    return out;
-  }
-
-  SavedVariable x, mean, rstd, w;
-  int64_t groups = 0;
-  bool has_w = false, has_b = false;
-};
-
-// y of a tensor that one rank holds whole, or None
-py::object gn_apply(const at::Tensor& x, int64_t groups, const c10::optional<at::Tensor>& w, const c10::optional<at::Tensor>& b, double eps,
-                    uintptr_t stream) {
-  if (any_tangent(x, w, b)) return py::none();
-  const bool grad = torch::autograd::compute_requires_grad(x, given(w), given(b));
-  at::Tensor y, kept, mean, rstd;
-  if (!gn_output(x, groups, w, b, eps, grad, stream, y, kept, mean, rstd)) return py::none();
-  if (grad) {
-    const auto node = node_of<GroupNormNode>(x, given(w), given(b));
-    node->x = SavedVariable(kept, false);
-    node->mean = SavedVariable(mean, false);
-    node->rstd = SavedVariable(rstd, false);
-    if (w) node->w = SavedVariable(*w, false);
-    node->groups = groups;
-    node->has_w = w.has_value();
-    node->has_b = b.has_value();
-    torch::autograd::set_history(y, node);
-  }
-  return py::cast(y);
-}
-
-struct LayerNormNode : Node {
-  std::string name() const override { return "_LayerNormBackward"; }
-  void release_variables() override {
-    const std::lock_guard<std::mutex> lock(mutex_);
-    for (SavedVariable* v : {&x_norm, &w, &std}) v->reset_data();
-  }
-  variable_list apply(variable_list&& grads) override {
-    variable_list out(3);
-    if (!grads[0].defined()) return out;
-    at::Tensor x_norm_, w_, std_;
-    {
-      const std::lock_guard<std::mutex> lock(mutex_);
-      x_norm_ = x_norm.unpack();
-      w_ = w.unpack();
-      std_ = std.unpack();
-    }
-    // hooks of the saved tensors may have given them another layout
-    x_norm_ = x_norm_.contiguous(), w_ = w_.contiguous(), std_ = std_.contiguous();
-    const at::Tensor g = grads[0].contiguous();
-    const uintptr_t stream = current_stream(g);
-    at::Tensor mean, dot;
-    const bool done = ln_sums(g, x_norm_, w_, std_, should_compute_output(1), should_compute_output(2), x_norm_.scalar_type(), stream, mean, dot, out[1], out[2]);
-    TORCH_CHECK(done, "layer_norm: what the backward got is not what the forward saved");
-    if (!should_compute_output(0)) return out;
-    if (ranks > 1) {
-      const py::gil_scoped_acquire gil;
-      try {
-        reduce.get()(mean, "avg", group.get());
-        reduce.get()(dot, "sum", group.get());
-      } catch (py::error_already_set& e) {
-        raise_as_is(e);
-      }
-    }
-    out[0] = ln_bwd_apply(g, x_norm_, w_, mean, dot, std_, x_norm_.size(-1) * ranks, stream).to(in_type);
-    return out;
-  }
-
-  SavedVariable x_norm, w, std;
-  Held reduce, group;
-  int64_t ranks = 1;
-  at::ScalarType in_type = at::kFloat;
-};
-
-// y from the statistics, with the node behind it where a gradient is wanted. `reduce(t, "avg" | "sum", group)` adds t up over the ranks.
-at::Tensor ln_output(const at::Tensor& x, const at::Tensor& mean, const at::Tensor& var, const at::Tensor& std, const at::Tensor& w,
-                     const c10::optional<at::Tensor>& b, double eps, const py::object& reduce, const py::object& group, int64_t ranks, uintptr_t stream) {
-  at::Tensor y, x_norm, var_eps;
-  ln_normalise(x, mean, var, std, w, b, eps, stream, y, x_norm, var_eps);
-  if (torch::autograd::compute_requires_grad(x, w, given(b))) {
-    const auto node = node_of<LayerNormNode>(x, w, given(b));
-    node->x_norm = SavedVariable(x_norm, false);
-    node->w = SavedVariable(w, false);
-    node->std = SavedVariable(std, false);
-    if (ranks > 1) {
-      node->reduce.hold(reduce);
-      node->group.hold(group);
-    }
-    node->ranks = ranks;
-    node->in_type = x.scalar_type();
-    torch::autograd::set_history(y, node);
-  }
-  return y;
-}
-// Whether ln_output takes these: parameters in the type that y gets, nothing to be copied, no tangents
-bool ln_takes(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& b, const at::ScalarType type) {
-  auto parameter = [&](const at::Tensor& t) {
-    return on_gpu(t) && t.scalar_type() == type && t.device() == x.device() && t.dim() == 1 && t.size(0) == x.size(-1);
-  };
-  return x.dim() >= 1 && x.numel() > 0 && on_gpu(x) && code_of(x) >= 0 && parameter(w) && code_of(w) >= 0 && (!b || parameter(*b)) && !any_tangent(x, w, b);
 }
 
 // ---- projections around attention and the Swin block: the launches of projection.py and swin._WholeBlock in their order, for
@@ -896,58 +600,6 @@ py::object projection_backward(const at::Tensor& g, const at::Tensor& x, const a
   return py::make_tuple(given(gx, need_x), given(gw, need_w), given(gb, need_b));
 }
 
-struct ProjectionNode : Node {
-  std::string name() const override { return qkv ? "_QkvProjectionBackward" : "_HeadsProjectionBackward"; }
-  void release_variables() override {
-    const std::lock_guard<std::mutex> lock(mutex_);
-    x.reset_data();
-    w.reset_data();
-  }
-  variable_list apply(variable_list&& grads) override {
-    variable_list out(3);
-    const at::Tensor g = defined_or_zeros(*this, grads[0]).contiguous();
-    at::Tensor x_, w_;
-    {
-      const std::lock_guard<std::mutex> lock(mutex_);
-      x_ = x.unpack();
-      w_ = w.unpack();
-    }
-    // hooks of the saved tensors may have given them another layout
-    x_ = x_.contiguous(), w_ = w_.contiguous();
-    const py::gil_scoped_acquire gil;
-    try {
-      // by its name in the module, as the Python route calls it
-      const py::object done = py::module_::import("jigsaw_amd._host").attr("projection_backward")(
-          g, x_, w_, qkv, l.b, l.h, l.s, l.d, should_compute_output(0), should_compute_output(1), should_compute_output(2), current_stream(g));
-      TORCH_CHECK(!done.is_none(), "projection: what the backward got is not what the forward saved");
-      const py::tuple all = done;
-      for (size_t i = 0; i < 3; ++i)
-        if (!all[i].is_none()) out[i] = all[i].cast<at::Tensor>();
-    } catch (py::error_already_set& e) {
-      raise_as_is(e);
-    }
-    return out;
-  }
-
-  SavedVariable x, w;
-  Heads l;
-  bool qkv = false;
-};
-
-// Whether nothing but autograd's graph stands between a forward of above and its result: no tangents
-bool projection_takes(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& b) { return !any_tangent(x, w, b); }
-// Puts the node behind the output y of either, where a gradient is wanted
-void projection_node(const at::Tensor& y, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& b, bool qkv) {
-  if (!torch::autograd::compute_requires_grad(x, w, given(b))) return;
-  const at::Tensor& split = qkv ? y : x;
-  const auto node = node_of<ProjectionNode>(x, w, given(b));
-  node->x = SavedVariable(x, false);
-  node->w = SavedVariable(w, false);
-  node->l = {split.numel() / ((qkv ? 3 : 1) * split.size(-1) * split.size(-2) * split.size(-3)), split.size(-3), split.size(-2), split.size(-1)};
-  node->qkv = qkv;
-  torch::autograd::set_history(y, node);
-}
-
 // One pass of swin._WholeBlock with bf16 tokens and fp32 parameters on a grid that wraps inside the rank: what its backward reads.
 // The block's parameters in the order of swin._WholeBlock.forward.
 enum Param { N1W, N1B, QKV_W, QKV_B, TABLE, PROJ_W, PROJ_B, N2W, N2B, FC1_W, FC1_B, FC2_W, FC2_B, PARAMS };
@@ -1000,16 +652,8 @@ class SwinPass {
   // 65536 tokens of 128 channels and 68 at 262144 of 256, 279 and 1879 with all of it kept until the end (136 and 1080 through
   // Python), and the memory that comes back at once is still in the caches (the first step 441 -> 427 us). The pass keeps nothing afterwards.
   py::object backward(const at::Tensor& grad, bool need_x, uintptr_t stream) {
-    List g;
-    if (!gradients(grad, need_x, stream, g)) return py::none();
-    py::tuple all(1 + PARAMS);
-    for (int i = 0; i <= PARAMS; ++i) all[i] = g[i].defined() ? py::cast(g[i]) : py::none();
-    return std::move(all);
-  }
-  // `backward` as tensors; false: declined
-  bool gradients(const at::Tensor& grad, bool need_x, uintptr_t stream, List& all) {
     if (!x.defined() || grad.sizes() != x.sizes() || !on_gpu(grad) || !aligned(grad) || grad.scalar_type() != at::kBFloat16 || grad.device() != x.device())
-      return false;
+      return py::none();
     at::AutoDispatchBelowADInplaceOrView below;
     void* const s = pointer(stream);
     const int64_t c = x.size(3), rows = l.b * l.s, hidden = pre.size(3);
@@ -1050,10 +694,11 @@ class SwinPass {
     drop(dqkv, y1);
     const at::Tensor gx = norm_backward(gy, gx1, x, mean1, rstd1, n1w, need_x, &g[N1W], &g[N1B], later, s);
     check(jg_reduce_many(&later.sums, s), "jg_reduce_many");
-    all = {gx};
-    all.insert(all.end(), g, g + PARAMS);
+    py::tuple all(1 + PARAMS);
+    all[0] = need_x ? py::cast(gx) : py::none();
+    for (int i = 0; i < PARAMS; ++i) all[1 + i] = py::cast(g[i]);
     *this = SwinPass();
-    return true;
+    return std::move(all);
   }
 
  private:
@@ -1115,75 +760,15 @@ class SwinPass {
   int64_t h = 0, w = 0, shift = 0;
 };
 
-struct SwinNode : Node {
-  std::string name() const override { return "_WholeBlockBackward"; }
-  void release_variables() override {
-    const std::lock_guard<std::mutex> lock(mutex_);
-    pass.reset();
-  }
-  variable_list apply(variable_list&& grads) override {
-    std::unique_ptr<SwinPass> taken;
-    {
-      const std::lock_guard<std::mutex> lock(mutex_);
-      taken = std::move(pass);
-    }
-    TORCH_CHECK(taken != nullptr,
-                "SwinBlock (one autograd node): backward was called a second time, but the tensors the first pass kept were released when it finished "
-                "(they are not held through save_for_backward, so retain_graph=True does not keep them). Run the forward again, or build the block with "
-                "one_node=False.");
-    at::Tensor g = defined_or_zeros(*this, grads[0]).contiguous();
-    if (!aligned(g)) g = g.clone();
-    variable_list out;
-    const bool done = taken->gradients(g, should_compute_output(0), current_stream(g), out);
-    TORCH_CHECK(done, "SwinBlock (one autograd node): the gradient is not of the output's shape and type");
-    return out;
-  }
-
-  std::unique_ptr<SwinPass> pass;
-};
-
-// Whether a native node may stand for the block: all parameters want a gradient or nothing does, and there are no tangents
-bool swin_takes(const at::Tensor& x, const List& p) {
-  bool all = true, any = torch::autograd::compute_requires_grad(x);
-  for (const at::Tensor& t : p) {
-    const bool wants = torch::autograd::compute_requires_grad(t);
-    all &= wants, any |= wants;
-    if (has_tangent(t)) return false;
-  }
-  return (all || !any) && !has_tangent(x);
-}
-// Puts the node behind the result y of `swin_forward`, where a gradient is wanted
-void swin_node(const at::Tensor& y, SwinPass& pass, const at::Tensor& x, const List& p) {
-  List inputs{x};
-  inputs.insert(inputs.end(), p.begin(), p.end());
-  if (!torch::autograd::compute_requires_grad(inputs)) return;
-  std::shared_ptr<SwinNode> node(new SwinNode(), torch::autograd::deleteNode);
-  node->set_next_edges(torch::autograd::collect_next_edges(inputs));
-  node->pass = std::make_unique<SwinPass>(std::move(pass));
-  torch::autograd::set_history(y, node);
-}
-
-// The Python type of a node's `grad_fn`
-template <typename N>
-void name_node(const char* name) {
-  static PyTypeObject type;
-  torch::autograd::_initFunctionPyTypeObject(type, name, nullptr, nullptr);
-  torch::autograd::registerCppFunction(typeid(N), &type);
-}
-
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  name_node<ConvNode>("_ConvNdBackward");
-  name_node<LayerNormNode>("_LayerNormBackward");
-  name_node<GroupNormNode>("_GroupNormOutputBackward");
-  name_node<ProjectionNode>("_ProjectionBackward");
-  name_node<SwinNode>("_WholeBlockBackward");
   py::class_<SumsLeft>(m, "SumsLeft");
   py::class_<Step>(m, "Step")
       .def(py::init<const py::tuple&, const py::tuple&, const py::tuple&, const py::tuple&, int, int, uintptr_t, uintptr_t, bool,
                     uintptr_t, const std::vector<size_t>&, const py::list&, const py::list&, const py::list&, const py::list&, bool>())
       .def_property_readonly("sends", &Step::sends)
+      .def("takes", &Step::takes)
       .def("pack", &Step::pack)
       .def("forward", &Step::forward)
       .def("backward", &Step::backward)
@@ -1193,16 +778,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("ring_forward_at_own_width", &ring_forward<true>);
   m.def("ring_backward", &ring_backward<false>);
   m.def("ring_backward_at_own_width", &ring_backward<true>);
+  m.def("ln_takes", &ln_takes);
   m.def("ln_partial", &ln_partial);
   m.def("ln_recentre", &ln_recentre);
   m.def("ln_apply", &ln_apply);
   m.def("ln_partial_bwd", &ln_partial_bwd);
   m.def("ln_bwd_apply", &ln_bwd_apply);
-  m.def("conv_takes", &conv_takes);
-  m.def("conv_apply", torch::wrap_pybind_function(conv_apply));
-  m.def("ln_takes", &ln_takes);
-  m.def("ln_output", torch::wrap_pybind_function(ln_output));
-  m.def("gn_apply", torch::wrap_pybind_function(gn_apply));
   m.def("gn_forward", &gn_forward);
   m.def("gn_backward", &gn_backward);
   m.def("qkv_forward", &qkv_forward);
@@ -1210,8 +791,4 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("projection_backward", &projection_backward);
   py::class_<SwinPass>(m, "SwinPass").def("backward", &SwinPass::backward);
   m.def("swin_forward", &SwinPass::forward);
-  m.def("projection_takes", &projection_takes);
-  m.def("projection_node", torch::wrap_pybind_function(projection_node));
-  m.def("swin_takes", &swin_takes);
-  m.def("swin_node", &swin_node);
 }

@@ -19,7 +19,7 @@ import torch
 import torch.distributed as dist
 
 from . import _lib
-from ._autograd import native_nodes
+from ._autograd import NativeFunction, native_nodes, saved_rows, wants_grad
 
 
 def _all_reduce_sum(t: torch.Tensor, groups: Sequence[Any]) -> None:
@@ -261,6 +261,21 @@ class _GroupNormOutput(torch.autograd.Function):
         return gx, None, None if gw is None else gw.to(dt_w), None if gb is None else gb.to(dt_b), None, None, None
 
 
+class _NativeGroupNormOutput(NativeFunction):
+    """``_GroupNormOutput`` of a tensor that one rank holds whole, in the type that it is computed in, by the native host
+    module: the same launches, less of the host."""
+
+    @staticmethod
+    def backward(ctx, g):  # noqa: D102
+        x, mean, rstd, w = saved_rows(ctx)
+        groups, grad_dtype = ctx.rest
+        got = _lib.host().gn_backward(g.to(x.dtype).contiguous(), x, mean, rstd, w, groups, *ctx.needs_input_grad[3:], grad_dtype,
+                                      _lib.stream_handle(g.device))
+        if got is None:
+            raise RuntimeError("group_norm: what the backward got is not what the forward saved")
+        return None, None, None, *got
+
+
 def group_norm(x, num_groups, weight=None, bias=None, spatial_groups=(), eps=1e-5):
     """``_GroupNorm.apply(...)[0]``, the call of ``DistributedGroupNorm.forward``, without the tensors only its other
     results need."""
@@ -271,10 +286,12 @@ def group_norm(x, num_groups, weight=None, bias=None, spatial_groups=(), eps=1e-
         return _GroupNorm.apply(x, num_groups, weight, bias, spatial_groups, eps)[0]
     split = tuple(g for g in spatial_groups or () if g is not None and int(g.size()) > 1)
     host = None if split or _compute_dtype(x) != x.dtype else _lib.host()
-    if host is not None and native_nodes():  # _GroupNormOutput without its Python
-        y = host.gn_apply(x, num_groups, weight, bias, float(eps), _lib.stream_handle(x.device))
-        if y is not None:
-            return y
+    if host is not None and native_nodes():
+        grad = wants_grad(x, weight, bias)
+        done = host.gn_forward(x, num_groups, weight, bias, float(eps), grad, _lib.stream_handle(x.device))
+        if done is not None:
+            y, kept, mean, rstd = done
+            return _NativeGroupNormOutput.apply(y, (kept, mean, rstd, weight), (num_groups, x.dtype), x, weight, bias) if grad else y
     return _GroupNormOutput.apply(x, num_groups, weight, bias, split, eps, torch.is_grad_enabled())
 
 

@@ -25,7 +25,7 @@ import math
 import torch
 
 from . import _lib
-from ._autograd import native_nodes
+from ._autograd import saved_rows
 
 
 def _nt(out, a, w, bias, rows, n_out, k_in, a_heads, out_heads, dims) -> None:
@@ -190,18 +190,6 @@ def _native(*tensors):
     return _lib.host() if all(t is None or (t.is_cuda and t.dtype == tensors[0].dtype) for t in tensors) else None
 
 
-def _native_apply(x, weight, bias, heads: int | None):
-    """The qkv projection, or the heads projection where ``heads`` is ``None``, with its autograd node in the native host module, or ``None``."""
-    host = _native(x, weight, bias) if not _remember_casts and native_nodes() else None
-    if host is None or not host.projection_takes(x, weight, bias):
-        return None
-    stream = _lib.stream_handle(x.device)
-    y = host.heads_forward(x, weight, bias, stream) if heads is None else host.qkv_forward(x, weight, bias, heads, stream)
-    if y is not None:
-        host.projection_node(y, x, weight, bias, heads is not None)
-    return y
-
-
 def _native_backward(ctx, grad, x, w, qkv: bool):
     """``(gx, gw, gb)`` from the native host module for a pass whose forward it ran, or ``None``; a pass whose weights came
     with their transposes (:func:`cast_parameters`) has fp32 parameters, which the native call does not know."""
@@ -250,7 +238,7 @@ class _QkvProjection(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad):  # noqa: D102
-        xc, w = ctx.saved_tensors
+        xc, w = saved_rows(ctx)
         got = _native_backward(ctx, grad, xc, w, True)
         if got is not None:
             return (*got, None)
@@ -319,7 +307,7 @@ class _HeadsProjection(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad):  # noqa: D102
-        oc, w = ctx.saved_tensors
+        oc, w = saved_rows(ctx)
         got = _native_backward(ctx, grad, oc, w, False)
         if got is not None:
             return (*got, None)
@@ -483,18 +471,12 @@ def gelu_mlp(x, w1, b1, w2, b2, residual=None):
 def qkv_projection(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, heads: int) -> torch.Tensor:
     """``rearrange(F.linear(x, weight, bias), "... s (three h d) -> three ... h s d", three=3, h=heads)``
     without the intermediate ``(..., s, 3 h d)`` tensor (_attention.py:881-890)."""
-    y = _native_apply(x, weight, bias, heads)
-    if y is not None:
-        return y
     return _QkvProjection.apply(x, weight, bias, heads)
 
 
 def heads_projection(out: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """``F.linear(rearrange(out, "... h s d -> ... s (h d)"), weight, bias)`` without the
     contiguous copy of the rearranged tensor (_attention.py:909-916)."""
-    y = _native_apply(out, weight, bias, None)
-    if y is not None:
-        return y
     return _HeadsProjection.apply(out, weight, bias, None)
 
 

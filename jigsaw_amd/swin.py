@@ -20,7 +20,6 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from ._autograd import native_nodes
 from .attention import _SwinGridAttention, swin_grid_attention_packed, window_attention
 from .conv import TileGroup
 from .layernorm import _PlainLayerNormFork, plain_layer_norm, plain_layer_norm_fork
@@ -392,15 +391,9 @@ class SwinBlock(nn.Module):
         dt = _compute_dtype(x)
         if self._one_node(x):
             attn, fc1, fc2 = self.attn, self.mlp[0], self.mlp[2]
-            params = (self.norm1.weight, self.norm1.bias, attn.qkv.weight, attn.qkv.bias, attn.bias_table, attn.proj.weight, attn.proj.bias,
-                      self.norm2.weight, self.norm2.bias, fc1.weight, fc1.bias, fc2.weight, fc2.bias)
-            host = _lib.host() if (not self.shift_by or self.shift_is_local()) and not casts_remembered() and native_nodes() else None
-            if host is not None and all(p is not None for p in params) and host.swin_takes(x, params):  # _WholeBlock without its Python
-                got = host.swin_forward(x, params, attn.side, attn.heads, self.shift_by, self.eps, _lib.stream_handle(x.device))
-                if got is not None:
-                    host.swin_node(*got, x, params)
-                    return got[0]
-            return _WholeBlock.apply(x, *params, self)
+            return _WholeBlock.apply(x, self.norm1.weight, self.norm1.bias, attn.qkv.weight, attn.qkv.bias, attn.bias_table,
+                                     attn.proj.weight, attn.proj.bias, self.norm2.weight, self.norm2.bias, fc1.weight, fc1.bias,
+                                     fc2.weight, fc2.bias, self)
         y, x = plain_layer_norm_fork(x, self.norm1.weight, self.norm1.bias, self.eps, out_dtype=dt)
         if self.attn.on_grid(y) and (not self.shift_by or self.shift_is_local()):
             b, h, w, c = x.shape

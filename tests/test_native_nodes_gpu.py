@@ -1,6 +1,9 @@
-"""Autograd nodes of the native host module (``csrc/host.cpp``) against the Python functions they stand for."""
+"""Autograd nodes behind results of the native host module (``_autograd.NativeFunction``) against the functions they stand for, and what
+autograd asks of the node of any layer."""
 
+import gc
 import itertools
+import weakref
 
 import pytest
 import torch
@@ -33,8 +36,9 @@ class Half:  # a channel group of two whose other half is the same rows
             t.mul_(2)
 
 
-def layer(kind, dev, back=None):
+def layer(kind, dev, back=None, group=None):
     """(call, differentiable tensors, name of the node) of one layer; its input first, its weight second."""
+    group = group or Half()
     gen = torch.Generator(device=dev).manual_seed(3)
     rand = lambda *shape: torch.randn(*shape, device=dev, generator=gen).bfloat16()  # noqa: E731
     if kind == "conv":
@@ -46,7 +50,7 @@ def layer(kind, dev, back=None):
         groups = (conv.TileGroup(3, 1),) * 2
         return (lambda x, w, b: conv._ConvNd.apply(x, w, b, one, one, one, groups, None, cfg)[0]), leaves, "ConvNd"
     if kind == "layernorm":
-        return (lambda x, w, b: layernorm.layer_norm(x, w, b, Half())), [rand(5, 7, 72), rand(72), rand(72)], "LayerNorm"
+        return (lambda x, w, b: layernorm.layer_norm(x, w, b, group)), [rand(5, 7, 72), rand(72), rand(72)], "LayerNorm"
     if kind == "groupnorm":
         return (lambda x, w, b: groupnorm.group_norm(x, 3, w, b)), [rand(2, 12, 9, 11), rand(12), rand(12)], "GroupNorm"
     if kind == "qkv":
@@ -64,13 +68,18 @@ def layer(kind, dev, back=None):
     return call, [rand(1, 16, 24, 64), *(p.detach().clone() for p in block.parameters())], "WholeBlock"
 
 
-KINDS = ["conv", "layernorm", "groupnorm", "qkv", "heads", "swin"]
+NATIVE = ["conv", "layernorm", "groupnorm"]
+KINDS = [*NATIVE, "qkv", "heads", "swin"]
+
+
+def is_native(y):
+    return issubclass(type(y.grad_fn)._forward_cls, _autograd.NativeFunction)
 
 
 def steps(kind, dev, need, monkeypatch, native, hooks=False):
     call, leaves, name = layer(kind, dev)
     if not native:
-        for module in (conv, layernorm, groupnorm, projection, swin):
+        for module in (conv, layernorm, groupnorm):
             monkeypatch.setattr(module, "native_nodes", lambda: False)
     leaves = [t.clone().requires_grad_(need[min(i, 1)]) for i, t in enumerate(leaves)]
     packed = []
@@ -89,16 +98,16 @@ def steps(kind, dev, need, monkeypatch, native, hooks=False):
             assert torch.equal(a, b)
     with pytest.raises(RuntimeError, match="second time"):
         torch.autograd.grad(y, wanted, g)
-    return [y.detach(), *once], isinstance(y.grad_fn, torch.autograd.function.BackwardCFunction), packed
+    return [y.detach(), *once], is_native(y), packed
 
 
 @pytest.mark.parametrize("need", [(True, True), (True, False), (False, True)])
-@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("kind", NATIVE)
 def test_a_native_node_has_the_bits_of_the_python_function(kind, need, dev, monkeypatch):
-    here, python, _ = steps(kind, dev, need, monkeypatch, True)
-    assert python == (kind == "swin" and need == (True, False))  # frozen parameters: the block's parts skip their gradients
-    want, python, _ = steps(kind, dev, need, monkeypatch, False)
-    assert python
+    here, native, _ = steps(kind, dev, need, monkeypatch, True)
+    assert native
+    want, native, _ = steps(kind, dev, need, monkeypatch, False)
+    assert not native
     for a, b in zip(here, want, strict=True):
         assert a.dtype == b.dtype and torch.equal(a, b)
 
@@ -136,7 +145,7 @@ def test_what_a_native_node_refuses(kind, dev):
 def test_an_exception_of_the_exchange_arrives_as_it_was_raised(dev):
     call, leaves, _ = layer("conv", dev, back=KeyError("a strip that never came"))
     y = call(*(t.requires_grad_() for t in leaves))
-    assert not isinstance(y.grad_fn, torch.autograd.function.BackwardCFunction)
+    assert is_native(y)
     with pytest.raises(KeyError, match="a strip that never came"):
         y.sum().backward()
 
@@ -156,3 +165,34 @@ def test_strips_in_another_layout_take_the_python_route(way, dev, monkeypatch):
     assert _lib.host() is not None
     for a, b in zip(*results, strict=True):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_graph_built_eagerly_runs_backward_under_compiled_autograd(kind, dev):
+    from torch._dynamo import compiled_autograd
+
+    call, leaves, _ = layer(kind, dev)
+    y = call(*(t.requires_grad_() for t in leaves))
+    g = torch.randn(y.shape, device=dev, generator=torch.Generator(device=dev).manual_seed(8)).to(y.dtype)
+    want = torch.autograd.grad(y, leaves, g)
+    for _ in range(2):  # recorded, and again from the record
+        y = call(*leaves)
+        for t in leaves:
+            t.grad = None
+        with compiled_autograd._enable(lambda graph: graph):
+            y.backward(g)
+        for t, v in zip(leaves, want, strict=True):
+            assert torch.equal(t.grad, v)
+
+
+@pytest.mark.parametrize("kind", ["conv", "layernorm"])
+def test_the_collector_frees_a_result_that_its_exchange_keeps(kind, dev):
+    group = Half()
+    call, leaves, _ = layer(kind, dev, group=group)
+    keeper = call.__closure__[[c for c in call.__code__.co_freevars].index("cfg")].cell_contents.halo_exchange if kind == "conv" else group
+    keeper.kept = call(*(t.requires_grad_() for t in leaves))
+    assert is_native(keeper.kept)
+    gone = weakref.ref(keeper)
+    del call, leaves, group, keeper
+    gc.collect()
+    assert gone() is None
