@@ -89,7 +89,7 @@ struct TileRegs {
 };
 
 // 32 rows of a row-major matrix of row length d <= D to registers; rows from `rows` on and columns from d on become zero on their way to LDS.
-// They are read from the last row and piece there is: a load under a condition is waited for where the paths meet, on the spot (24 heads x
+// (REPEAT: such rows are the last row there is.) They are read from the last row and piece there is: a load under a condition is waited for where the paths meet, on the spot (24 heads x
 // 739 x 5 chunks, head size 32: forward 63 -> 48 us, dQ 54 -> 46). tid: thread of the group; at least one row lies before `rows`.
 template <int D, int W>
 __device__ __forceinline__ void tile_fetch(TileRegs<D, W>& r, const uint16_t* src, int tid, int rows, int d) {
@@ -100,14 +100,14 @@ __device__ __forceinline__ void tile_fetch(TileRegs<D, W>& r, const uint16_t* sr
     r.v[i] = *reinterpret_cast<const u32x4*>(src + min(c / (D / 8), rows - 1) * d + min(c % (D / 8) * 8, d - 8));
   }
 }
-template <int D, int W>
+template <int D, int W, bool REPEAT = false>
 __device__ __forceinline__ void tile_store(const TileRegs<D, W>& r, unsigned char* dst, int tid, int d) {
 #pragma unroll
   for (int i = 0; i < TileRegs<D, W>::PER; ++i) {
     const int c = tid + i * (W * 64);
     if (c < Geo<D>::CHUNKS) {
       const int row = c / (D / 8), piece = c % (D / 8);
-      const bool there = row < r.rows && piece * 8 < d;
+      const bool there = (REPEAT || row < r.rows) && piece * 8 < d;
       u32x4 v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = there ? r.v[i][e] : 0u;
@@ -791,7 +791,9 @@ __device__ __forceinline__ void dkv_block(const Args& p, const BlockOf& wg) {
   };
   auto store = [&](int buf) {
     unsigned char* base = lds + buf * BUF;
-    tile_store<D, W>(rq, base, tid, p.d);
+    // A query past the end is the last one once more, whose score less an lse of +inf is -inf: a row of zeros makes NaN of an infinite key, and
+    // NaN no probability of 0. (dO's row is zeros: what a probability that parts8 keeps above 0 is multiplied by.)
+    tile_store<D, W, true>(rq, base, tid, p.d);
     tile_store<D, W>(rg, base + G::TILE, tid, p.d);
     if (tid < 2 * BT) {
       float v = tid < BT ? st * LOG2E : st;

@@ -518,6 +518,33 @@ def test_a_chunk_without_a_finite_score_weighs_nothing_step_by_step(b, d, dtype,
         assert out[0].isnan().all() and lse[0].isnan().all() and not out[1:].isnan().any() and not lse[1:].isnan().any()
 
 
+@pytest.mark.parametrize("dtype,bar", [(torch.float32, 1e-5), (torch.bfloat16, 4e-3), (torch.float16, 5e-4)], ids=str)
+@pytest.mark.parametrize("b,sq,sk,d,P", [
+    # one launch: groups without a tile, one row in the last tile, chunks of fewer than 128 keys, workgroups of 32, 64 and 128 rows
+    (3, 33, 130, 64, 2), (3, 1, 150, 64, 1), (3, 70, 70, 32, 2), (71, 132, 95, 24, 3), (68, 80, 141, 32, 1), (5, 66, 150, 96, 1), (13, 102, 130, 128, 2),
+    # two launches, of both kernels of heads of 64
+    (18, 1000, 300, 64, 2), (300, 70, 140, 64, 1), (80, 300, 150, 32, 4), (60, 200, 200, 96, 2), (60, 200, 100, 128, 2), (3, 128, 128, 64, 2),
+])
+def test_keys_without_a_finite_score_get_no_gradient(b, sq, sk, d, P, dtype, bar, dev):
+    """dK and dV of keys whose scores are all -inf are 0, and the others' are those of the formula, against float64 (tolerances as
+    in :func:`test_backward_in_one_launch`; dQ is NaN by the formula: 0 x -inf). A whole block of dead keys and single ones. No
+    query is 0, which makes a score of NaN. A probability that is kept in three bf16 parts is 2^-126 where it is 0."""
+    gen = torch.Generator().manual_seed(b + sq)
+    q, g = (torch.randn(1, b, sq, d, generator=gen).abs() + 0.01).to(dtype), torch.randn(1, b, sq, d, generator=gen).to(dtype)
+    ks, vs = ([torch.randn(1, b, sk, d, generator=gen).to(dtype) for _ in range(P)] for _ in range(2))
+    dead = torch.zeros(sk, dtype=torch.bool)
+    dead[:32] = dead[sk - 1] = dead[sk // 2] = True
+    ks[0][..., dead, :] = float("-inf")
+    out, lse = ja.ring_forward(q.to(dev), [t.to(dev) for t in ks], [t.to(dev) for t in vs], d**-0.5)
+    _, dk, dv = ja.ring_backward(g.to(dev), q.to(dev), out, lse, [t.to(dev) for t in ks], [t.to(dev) for t in vs], d**-0.5)
+    k, v = torch.cat(ks, 2).double(), torch.cat(vs, 2).double()
+    _, wk, wv = oa.core_backward(g.double(), q.double(), k, v, out.cpu().double(), lse.cpu().double(), d**-0.5)
+    for got, want in ((dk, wk), (dv, wv)):
+        assert (got[0][..., dead, :].abs() <= sq * 2.0**-120).all()
+        got = torch.cat(got, 2).cpu().double()
+        assert (got - want).norm() <= bar * want.norm()
+
+
 @pytest.mark.parametrize("d,n,nk", [(64, 192, 160), (32, 100, 70), (128, 64, 96)])
 def test_fp32_ring_step_takes_the_fused_merge(d, n, nk, dev):
     """``attend_step_`` on fp32 tensors at the head sizes of the fp32 matrix-core kernel: one launch that merges in
