@@ -21,6 +21,7 @@ bool attn_mfma_bwd_supported(long long batch, int sq, int sk, int d, int dtype, 
 int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q,
                          const void* const* k, const void* const* v, int nchunks, const void* out, const float* lse,
                          long long batch, int sq, int sk, float scale, void* ws, hipStream_t s);
+int attn_mfma_bwd_one_launch_width(long long batch, int sq, int sk, int nchunks);
 bool attn_wide_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias);
 bool attn_f32_mfma_supported(long long batch, int sq, int sk, int d, int chunks, int dtype, bool has_bias);
 int attn_f32_mfma_fwd_chunks(void* out, float* lse, const void* q, const void* const* k, const void* const* v, int chunks,
@@ -213,4 +214,13 @@ extern "C" int jg_attn_bwd_chunks(void* dq, void* const* dk, void* const* dv, co
     return jg::attn_f32_mfma_bwd_chunks(dq, dk, dv, dout, q, k, v, (int)n_chunks, out, lse, batch, (int)sq, (int)sk, (int)d, scale,
                                         workspace, s);
   JG_FAIL(JG_ERR_UNSUPPORTED, "%s: bf16 or fp16, d a multiple of 8 up to 128, or fp32, d a multiple of 4 up to 128; 16-byte aligned tensors", who);
+}
+
+// Rows of a workgroup where jg_attn_bwd_chunks forms dQ, dK and dV of aligned tensors in one launch of attn_wide.hip, 0 where it does not: for
+// tests, which have to know what they reach, and not in the interface.
+extern "C" int jg_attn_bwd_one_launch_rows(int64_t n_chunks, int64_t batch, int64_t sq, int64_t sk, int64_t d, int dtype) {
+  if (check_shape("jg_attn_bwd_one_launch_rows", batch, sq, sk, d, 1.0f, dtype) != JG_OK) return 0;
+  if (jg::attn_mfma_bwd_supported(batch, (int)sq, (int)sk, (int)d, dtype, false)) return 32 * jg::attn_mfma_bwd_one_launch_width(batch, (int)sq, (int)sk, (int)n_chunks);
+  if (!jg::attn_wide_supported(batch, (int)sq, (int)sk, (int)d, dtype, false)) return 0;
+  return 32 * jg::attn_wide_bwd_one_launch_width(batch, (int)sq, (int)sk, (int)d, (int)n_chunks);
 }

@@ -596,6 +596,12 @@ bool attn_mfma_bwd_supported(long long batch, int sq, int sk, int d, int dtype, 
 
 // The ring backward over `nchunks` resident chunks: k[c], v[c] in, dk[c], dv[c] out, dq = the sum over
 // the chunks, rounded once. nchunks = 1 is the plain backward of one chunk.
+// Where bf16 heads of 64 go to attn_wide.hip for dQ, dK and dV in one launch: its rows of a workgroup / 32, else 0
+int attn_mfma_bwd_one_launch_width(long long batch, int sq, int sk, int nchunks) {
+  const bool ragged = sq % EXACT_KEYS != 0 || sk % EXACT_KEYS != 0;
+  return ragged && attn_width(sq, batch, D) == 1 ? attn_wide_bwd_one_launch_width(batch, sq, sk, D, nchunks) : 0;
+}
+
 int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q,
                          const void* const* k, const void* const* v, int nchunks, const void* out, const float* lse,
                          long long batch, int sq, int sk, float scale, void* ws, hipStream_t s) {
@@ -649,7 +655,7 @@ int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
   // chunks' number, as above.)
   const int width = attn_width(sq, batch, D);
   if (width == 1 || (width == 2 && (sq % EXACT_KEYS != 0 || sk % EXACT_KEYS != 0) && (long long)sk * nchunks >= 2048)) {
-    if (width == 1 && (sq % EXACT_KEYS != 0 || sk % EXACT_KEYS != 0) && attn_wide_bwd_one_launch(batch, sq, sk, nchunks))
+    if (attn_mfma_bwd_one_launch_width(batch, sq, sk, nchunks) != 0)
       return attn_wide_bwd_chunks(dq, dk, dv, dout, q, k, v, nchunks, out, lse, batch, sq, sk, D, JG_BF16, scale, ws, s);
     const int rc = attn_wide_bwd_chunks(dq, nullptr, nullptr, dout, q, k, v, nchunks, out, lse, batch, sq, sk, D, JG_BF16, scale, ws, s);
     if (rc != JG_OK) return rc;

@@ -99,7 +99,8 @@ int attn_wide_fwd_chunks(void* out, float* lse, const void* q, const void* const
 int attn_wide_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void* dout, const void* q, const void* const* k,
                          const void* const* v, int nchunks, const void* out, const float* lse, long long batch, int sq,
                          int sk, int d, int dtype, float scale, void* ws, hipStream_t s);
-bool attn_wide_bwd_one_launch(long long batch, int sq, int sk, int nchunks);  // whether that forms dQ, dK and dV of heads of 64 in one launch
+// Rows of a workgroup / 32 where that forms dQ, dK and dV in one launch, 0 where it takes two
+int attn_wide_bwd_one_launch_width(long long batch, int sq, int sk, int d, int nchunks);
 
 // Workgroup -> (batch entry, chunk, row block) of a grid (row blocks, batch entries, chunks). Consecutive
 // workgroup ids go to the 8 XCDs in turn; each XCD is given a contiguous range of the flat order (batch entry,

@@ -1057,7 +1057,9 @@ double steps_alone(long long workgroups, long long steps, int wavefronts) {
   const long long each = jg::cdiv(workgroups, jg::cu_count());
   return (wavefronts == 8 ? (each == 1 ? 1.8 : 2.0 * each) : (each == 1 ? 1.1 : 1.0 * each)) * steps;
 }
-// Rows a workgroup / 32 of the one launch (0: two launches)
+// Rows a workgroup / 32 of the one launch (0: two launches). Its workgroups lie in one dimension of the grid, which holds 2^32 threads: 2^24 workgroups of
+// 256. (Two launches have three dimensions. Rings of very many short heads come that far: 65535 x 64 queries against 16 x 1024 keys.)
+constexpr long long MOST_BLOCKS = (1ll << 24) - 1;
 template <int D>
 int one_launch_width(const Args& a, long long batch) {
   const int tq = jg::cdiv(a.sq, BT), tk = jg::cdiv(a.sk, BT);
@@ -1066,6 +1068,7 @@ int one_launch_width(const Args& a, long long batch) {
   auto blocks_k = [&](int w) { return jg::cdiv(tk, w) * batch * a.nchunks; };
   auto steps_q = [&](int ks) { return (long long)jg::cdiv((long long)tk * a.nchunks, ks); };
   auto steps_k = [&](int ks) { return (long long)jg::cdiv(tq, ks); };
+  auto fit = [&](int w) { return blocks_q(w) + blocks_k(w) <= MOST_BLOCKS; };
   const Shape q = dq_shape<D>(a, batch), k = dkv_shape<D>(a, batch);
   int width = 0;
   if (D <= 64) {
@@ -1073,7 +1076,7 @@ int one_launch_width(const Args& a, long long batch) {
     for (int w = 1; w <= 4; w *= 2) {
       const double load = double(blocks_q(w) * steps_q(4 / w) + blocks_k(w) * steps_k(4 / w)) / jg::cu_count();
       const double one = std::max(1.1 * std::max(steps_q(4 / w), steps_k(4 / w)), load * (w == 1 ? (D == 32 ? 1.2 : 1.7) : (D == 32 ? 1.0 : 1.25)));
-      if (one < least) least = one, width = w;
+      if (one < least && fit(w)) least = one, width = w;
     }
     return width;
   }
@@ -1096,7 +1099,6 @@ int launch_bwd(const ChunkTable& tab, const Args& a, long long batch, int width,
     constexpr int STAGES = KS * 2 * (2 * G::TILE + (1 + G::DOTS) * BT * 4), SUMS = KS / 2 * W * 16 * G::NB * 64 * 4, LDS = std::max(STAGES, SUMS);
     static_assert(LDS <= 160 * 1024, "fits LDS");
     const long long rq = jg::cdiv(a.sq, 32 * W), rk = jg::cdiv(a.sk, 32 * W), nq = rq * batch, nk = rk * batch * a.nchunks;
-    JG_REQUIRE(nq + nk < (1ll << 31), "%s: too many workgroups", who);
     constexpr auto kernel = &attn_wide_bwd_kernel<D, F16, W, EXACT>;
     if (LDS > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
       JG_FAIL(JG_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS", who, LDS);
@@ -1122,10 +1124,10 @@ int by_width(int d, int dtype, F f) {
 
 namespace jg {
 
-bool attn_wide_bwd_one_launch(long long batch, int sq, int sk, int nchunks) {
+int attn_wide_bwd_one_launch_width(long long batch, int sq, int sk, int d, int nchunks) {
   Args a{};
   a.sq = sq; a.sk = sk; a.nchunks = nchunks;
-  return one_launch_width<64>(a, batch) != 0;
+  return by_width(d, JG_BF16, [&](auto width, auto) { return one_launch_width<width()>(a, batch); });
 }
 
 bool attn_wide_supported(long long batch, int sq, int sk, int d, int dtype, bool has_bias) {
