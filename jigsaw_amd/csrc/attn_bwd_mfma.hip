@@ -648,7 +648,7 @@ int attn_mfma_bwd_chunks(void* dq, void* const* dk, void* const* dv, const void*
   // traffic and a barrier for half the keys cost more than the waves' independence gives: 8 x 4096 x 4 203 : 223, 32 x 1024 x 1
   // 18.0 : 18.9, 24 x 1000 x 2 30.8 : 32.1.
   // And there dQ, dK and dV in one launch where attn_wide.hip takes that to be the shorter way (two launches : one, us; fp16 for the latter): 7 x 387 x 6 chunks
-  // 35.2 : 27.3, 15 x 313 x 7 42.9 : 31.6, 6 x 400 x 4 25.8 : 20.2. (Not for lengths in multiples of 128, where dK and dV of a chunk have the same bits in a ring
+  // 35.2 : 27.3, 6 x 400 x 4 25.8 : 20.2. (Not for lengths in multiples of 128, where dK and dV of a chunk have the same bits in a ring
   // and by themselves: attention.backward_chunks.)
   // Those of 64 queries go there too where the keys are many (four groups take tiles of all chunks in turn; this kernel with 64 : that one, backward, us): 32 x 270 x 8
   // 55.8 : 51.1, 30 x 394 x 6 65.8 : 61.4, 48 x 237 x 6 41.9 : 40.2, 4 x 2700 x 5 217 : 202; 18 x 745 x 2 35.4 : 35.9, 27 x 296 x 2 21.4 : 21.9. (Lengths in multiples of 128: not by a rule on the

@@ -1045,10 +1045,10 @@ int launch_dkv(const ChunkTable& tab, const Args& a, long long batch, hipStream_
 // Up to 64 columns both ways are priced in steps of a workgroup of four wavefronts (about 0.45 us at 32 columns, 0.75 at 64): a compute unit makes
 // one at a time, 1.1 of them where it has a workgroup alone, and one of eight wavefronts takes 1.8 and 2. In one launch a head of 64 columns takes 1.25 (its
 // registers let two workgroups on a compute unit), and workgroups of 32 rows, which fetch a tile for one wavefront each, 1.2 and 1.7. A launch more is
-// six steps. Taken where one launch is expected to need less than 0.8 of the two. Backward, two launches : one, us: 4 heads x 128 x 2 chunks at 32
+// six steps. Taken where one launch is expected to need less than 0.8 of the two (0.72 up to 96 columns, 0.85 above: the rings below). Backward, two launches : one, us: 4 heads x 128 x 2 chunks at 32
 // 11.3 : 7.7, 15 x 710 x 3 at 32 38.6 : 24.2, 3 x 1497 x 2 at 32 30.1 : 20.4, 16 x 802 x 3 at 32 41.7 : 31.6, 3 x 3000 x 4 at 32 140 : 100, 64 x 64 x 1 at 64
-// 14.6 : 7.1, 48 x 69 x 3 at 64 22.0 : 14.2, 15 x 313 x 7, fp16 64 42.9 : 31.6, 7 x 387 x 6, fp16 64 36.5 : 27.3. Where it says no: 8 x 1024 x 8 at 32
-// 59.0 : 61.5, 24 x 1000 x 2, fp16 64 71.7 : 74.7.
+// 14.6 : 7.1, 48 x 69 x 3 at 64 22.0 : 14.2, 7 x 387 x 6, fp16 64 36.5 : 27.3. Where it says no: 8 x 1024 x 8 at 32
+// 59.0 : 61.5, 24 x 1000 x 2, fp16 64 71.7 : 74.7 (but 15 x 313 x 7, fp16 64 37.0 : 31.6, which it prices at 34 steps and 38).
 // Wider heads have one workgroup of the one launch on a compute unit: it is taken where all of them fit at once, priced in us by what a step took
 // there, by rows, with nine for a launch and what surrounds it. 13 x 102 x 2 at 128 21.8 : 12.7, 7 x 265 x 1 at 128 26.5 : 19.7, 2 x 2000 x 2 at 128
 // 119 : 93, 2 x 1000 x 3 at 96 52.3 : 33.0, 16 x 200 x 3 at 96 23.4 : 15.4, 40 x 90 x 4 at 80 27.4 : 19.2, 1 x 2500 x 2 at 96 92 : 66. Where it says no: 12 x 1180 x 1

@@ -11,6 +11,7 @@ import torch
 from helpers import rel_l2
 from jigsaw_amd import attention as ja
 from oracle import attention as oa
+from test_attention_routes import ONE_LAUNCH, one_launch_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -854,17 +855,12 @@ def test_narrow_heads_with_many_rows_keep_their_width(h, d, dev):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("h,sq,sk,d,P", [
-    # workgroups of 32, 64 and 128 rows on a chip of 256 compute units; chunks from 128 keys on and shorter ones
-    (10, 22, 130, 32, 1), (3, 24, 89, 24, 2), (68, 80, 141, 32, 1), (79, 37, 29, 8, 4), (78, 201, 252, 32, 1), (71, 132, 95, 24, 3),
-    (1, 59, 375, 64, 1), (2, 31, 89, 40, 2), (74, 22, 206, 64, 1), (56, 61, 27, 56, 1), (55, 203, 194, 64, 1), (57, 139, 88, 64, 2),
-    (4, 1, 300, 64, 2), (4, 300, 1, 32, 2),
-    # wider heads: the same three, where all workgroups fit at once
-    (5, 66, 70, 96, 1), (13, 102, 130, 128, 2), (3, 260, 200, 80, 3), (16, 200, 150, 96, 3), (2, 1000, 900, 128, 2), (40, 90, 100, 72, 4), (1, 500, 700, 120, 1),
-])
+@pytest.mark.parametrize("h,sq,sk,d,P", list(ONE_LAUNCH))
 def test_backward_in_one_launch(h, sq, sk, d, P, dtype, dev):
     """dQ, dK and dV of small rings, one launch with delta formed twice, against float64: one rounding to 16 bits of dS and P (none in short
     chunks) and one of the result, 2^-9 (bf16) and 2^-12 (fp16) each at most, of terms of both signs."""
+    if _compute_units() == 256:
+        assert one_launch_rows(h, sq, sk, d, P, dtype) == ONE_LAUNCH[h, sq, sk, d, P][dtype == torch.float16]
     gen = torch.Generator().manual_seed(h + sq)
     q, g = ((torch.randn(1, h, sq, d, generator=gen) * f).to(dtype) for f in (d**-0.5, 1.0))
     ks, vs = ([torch.randn(1, h, sk, d, generator=gen).to(dtype) for _ in range(P)] for _ in range(2))
