@@ -448,6 +448,7 @@ constexpr unsigned long long kEmpty = ~0ull;
 //   (for 20 ms) 1158 / 2508 : 2627 / 3956
 //   2 x 64 x 512^2, 2 groups      0   40 / 49 : 39 / 52      150   89 / 315 : 91 / 342       200   355 / 533 : 293 / 463
 constexpr unsigned kPolls = 128, kPollsStarved = 48;
+constexpr unsigned kOwnChoice = ~0u;  // for `polls`: as the interface has it, a whole group a block where that covers the tensor, else kPolls
 constexpr long long kStreamed = 1ll << 27;  // bytes of a tensor that goes past the last-level cache
 constexpr int kMaxPartials = 2 * kThreads;  // partials of a unit: every block of the unit adds them up again
 
@@ -942,9 +943,11 @@ bool resident_launch(ResidentArgs q, const ApplyArgs& a, void* gw, void* gb, int
   q.partials = (unsigned)(cpg * chunks);
   q.S = S;
   q.chunk_len = chunk_len_of(S, (int)chunks);
+  const bool own_choice = q.polls == kOwnChoice;
+  if (own_choice) q.polls = kPolls;
   const long long channels = gw != nullptr || gb != nullptr ? a.C : 0, bytes = rows * S * (long long)sizeof(typename Elem<DT>::T);
-  // A unit of up to kWhole chunks is one block's. (Not for `polls` of a test's own.)
-  if (q.partials <= kWhole && q.polls == kPolls && bytes < kStreamed) {
+  // A unit of up to kWhole chunks is one block's.
+  if (own_choice && q.partials <= kWhole && bytes < kStreamed) {
     gn_resident_kernel<DT, BWD, false, true><<<(unsigned)units, kThreads * q.partials, 0, s>>>(q, a);
     q.left = nullptr;
     if (channels > 0) gn_resident_rest_kernel<DT, BWD><<<(unsigned)channels, kThreads, 0, s>>>(q, a, gw, gb, wdtype, N);
@@ -1095,8 +1098,8 @@ int backward_all(void* gx, void* gw, void* gb, int wdtype, const void* g, const 
 }  // namespace
 
 // jg_gn_forward_keep and jg_gn_backward as they are but for `polls`: how often a block asks for the rest of its group before
-// it leaves its chunk to the second launch (1: nearly always; 0: separate launches, which read the tensors twice). Not in the
-// header: tests reach both launches through them.
+// it leaves its chunk to the second launch (1: nearly always; 0: separate launches, which read the tensors twice; kOwnChoice). Not
+// in the header: tests reach every launch through them.
 extern "C" int jg_gn_forward_polls(void* y, void* x_kept, float* mean, float* rstd, const void* x, const void* weight,
                                    const void* bias, int64_t batch, int64_t channels, int64_t spatial, int64_t groups,
                                    float eps, int dtype, unsigned polls, void* workspace, size_t workspace_bytes, void* stream);
@@ -1115,7 +1118,7 @@ extern "C" int jg_gn_forward(void* y, float* mean, float* rstd, const void* x, c
 extern "C" int jg_gn_forward_keep(void* y, void* x_kept, float* mean, float* rstd, const void* x, const void* weight,
                                   const void* bias, int64_t batch, int64_t channels, int64_t spatial, int64_t groups,
                                   float eps, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
-  return jg_gn_forward_polls(y, x_kept, mean, rstd, x, weight, bias, batch, channels, spatial, groups, eps, dtype, kPolls, workspace,
+  return jg_gn_forward_polls(y, x_kept, mean, rstd, x, weight, bias, batch, channels, spatial, groups, eps, dtype, kOwnChoice, workspace,
                              workspace_bytes, stream);
 }
 
@@ -1139,7 +1142,7 @@ extern "C" int jg_gn_backward(void* gx, void* gw, void* gb, const void* g, const
                               const float* rstd, const void* weight, int64_t batch, int64_t channels, int64_t spatial,
                               int64_t groups, int dtype, int grad_dtype, void* workspace, size_t workspace_bytes,
                               void* stream) {
-  return jg_gn_backward_polls(gx, gw, gb, g, x, mean, rstd, weight, batch, channels, spatial, groups, dtype, grad_dtype, kPolls,
+  return jg_gn_backward_polls(gx, gw, gb, g, x, mean, rstd, weight, batch, channels, spatial, groups, dtype, grad_dtype, kOwnChoice,
                               workspace, workspace_bytes, stream);
 }
 

@@ -214,7 +214,10 @@ def test_input_changed_in_place_before_the_backward(shape, dtype, sharded, dev):
     assert rel_l2(x, want) < TOL[dtype]
 
 
-@pytest.mark.parametrize("polls", [0, 1, 256])  # separate launches; nearly every chunk left to the second launch; hardly any
+OWN_CHOICE = 2**32 - 1  # for `polls`: what group_norm takes, a whole group a block where that covers the tensor
+
+
+@pytest.mark.parametrize("polls", [0, 1, 256, OWN_CHOICE])  # separate launches; nearly every chunk left to the second launch; hardly any; group_norm's
 @pytest.mark.parametrize("shape", [
     # batch, channels, groups, positions; a block keeps 16384 (backward) or 32768 (forward) 16-bit elements, half as many fp32
     (2, 6, 3, 1), (2, 6, 2, 7), (1, 8, 2, 4097), (1, 4, 2, 16384), (2, 4, 2, 16385), (1, 2, 1, 32777),
@@ -285,6 +288,7 @@ def _whole_tensor(shape, dtype, dev):
                                         _lib.dtype_code(grads.dtype), polls, p(ws), nbytes, stream) == 0
         return {"y": y, "kept": kept, "gx": gx, "stats": stats, "grads": grads}
 
+    run.x = x
     return run
 
 
@@ -311,11 +315,31 @@ def test_the_launch_that_writes_a_chunk_does_not_show(shape, dtype, dev):
 ], ids=str)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_a_group_that_one_block_keeps_has_the_bits_of_several(shape, dtype, dev):
-    """The default call (128 polls), where small groups meet in LDS, and the same with blocks that wait for each other."""
+    """What group_norm takes, where small groups meet in LDS, and the same with blocks that wait for each other."""
     run = _whole_tensor(shape, dtype, dev)
-    got, want = run(128), run(256)
+    got, want = run(OWN_CHOICE), run(256)
     for name, t in got.items():
         assert not t.isnan().any() and torch.equal(t, want[name]), name
+
+
+@pytest.mark.parametrize("shape", [(2, 8, 4, 1000), (1, 4, 2, 16384), (3, 4, 4, 40001)], ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_infinities_and_nan_stay_in_their_group(shape, dtype, dev):
+    """x with one infinity in the first group and one NaN in the last: those come out without a finite value, the others as without
+    them, and a block that keeps a whole group has the same results as blocks that wait for each other."""
+    N, C, G, S = shape
+    run = _whole_tensor(shape, dtype, dev)
+    clean = run(OWN_CHOICE)
+    run.x[0, 0, S // 2], run.x[N - 1, C - 1, S - 1] = float("inf"), float("nan")
+    got, want = run(OWN_CHOICE), run(256)
+    sick = torch.zeros(N, G, dtype=torch.bool, device=dev)
+    sick[0, 0] = sick[N - 1, G - 1] = True
+    for name in ("y", "kept", "gx", "stats"):
+        a, b, c = (t[name].permute(1, 2, 0) if name == "stats" else t[name].view(N, G, -1) for t in (got, want, clean))
+        assert torch.equal(a.nan_to_num(nan=7.0), b.nan_to_num(nan=7.0)) and torch.equal(a[~sick], c[~sick]), name
+        assert name == "kept" or not a[sick][..., :1].isfinite().any(), name
+    a, b = got["grads"], want["grads"]
+    assert torch.equal(a.nan_to_num(nan=7.0), b.nan_to_num(nan=7.0)) and a[1].isfinite().all()
 
 
 def test_a_busy_chip_does_not_show_in_the_results(dev):
