@@ -25,6 +25,7 @@ from collections.abc import Sequence
 import torch
 
 from . import _lib
+from ._autograd import saved_rows
 
 _SUPPORTED_O = (torch.float16, torch.bfloat16, torch.float32)
 
@@ -466,7 +467,7 @@ class _BiasedAttention(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out):  # noqa: D102
-        q, k, v, bias, out, lse = ctx.saved_tensors
+        q, k, v, bias, out, lse = saved_rows(ctx)
         need_bias = bias is not None and ctx.needs_input_grad[3]
         res = core_backward(grad_out, q, k, v, out, lse, ctx.scale, bias=bias, want_dbias=need_bias)
         dq, dk, dv = res[:3]
@@ -529,7 +530,7 @@ class _SwinGridAttention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out):  # noqa: D102
         lib = _lib.load()
-        qkv, table, side, out, lse = ctx.saved_tensors
+        qkv, table, side, out, lse = saved_rows(ctx)
         _, images, heads, tokens, d = qkv.shape
         gh, gw = ctx.grid
         grad_out = grad_out.contiguous()

@@ -140,7 +140,7 @@ class _GroupNorm(torch.autograd.Function):
     def backward(ctx, grad_output, x_norm_grad, rstd_grad, n_grad):  # noqa: D102
         if grad_output is None:
             return (None,) * 6
-        x_norm, rstd, count, w = ctx.saved_tensors
+        x_norm, rstd, count, w = saved_rows(ctx)
         g = grad_output.to(x_norm.dtype).contiguous()
         n, c, s = _dims(x_norm)
         groups = ctx.num_groups
@@ -220,7 +220,7 @@ class _GroupNormOutput(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):  # noqa: D102
-        x, mean, rstd, count, w = ctx.saved_tensors
+        x, mean, rstd, count, w = saved_rows(ctx)
         g = grad_output.to(x.dtype).contiguous()
         n, c, s = _dims(x)
         groups = ctx.num_groups

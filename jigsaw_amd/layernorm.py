@@ -150,7 +150,7 @@ class _LayerNorm(PositionalFunction):
     def backward(ctx, grad_output, x_norm_grad, weight_grad, var_grad):  # noqa: D102
         if grad_output is None:
             return (None,) * 5
-        x_norm, w, std = ctx.saved_tensors
+        x_norm, w, std = saved_rows(ctx)
         g = grad_output.to(x_norm.dtype).contiguous()
         group = ctx.channel_group
         cols = x_norm.shape[-1]
@@ -263,7 +263,7 @@ class _PlainLayerNorm(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad, past=None):  # noqa: D102
-        xc, mean, rstd, w = ctx.saved_tensors
+        xc, mean, rstd, w = saved_rows(ctx)
         cols = xc.shape[-1]
         rows = xc.numel() // cols
         g = grad.contiguous()

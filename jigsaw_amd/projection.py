@@ -356,7 +356,7 @@ class _Linear(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad):  # noqa: D102
-        xc, w = ctx.saved_tensors
+        xc, w = saved_rows(ctx)
         n_out, k = w.shape
         rows = xc.numel() // k
         g = grad.to(xc.dtype).contiguous()
@@ -432,7 +432,7 @@ class _GeluMlp(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad):  # noqa: D102
-        xc, pre, act, w1c, w2c = ctx.saved_tensors
+        xc, pre, act, w1c, w2c = saved_rows(ctx)
         hid, k = w1c.shape
         n_out = w2c.shape[0]
         rows = xc.numel() // k

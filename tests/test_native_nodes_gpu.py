@@ -8,7 +8,7 @@ import weakref
 import pytest
 import torch
 
-from jigsaw_amd import _autograd, _lib, conv, groupnorm, layernorm, projection, swin
+from jigsaw_amd import _autograd, _lib, attention, conv, groupnorm, layernorm, projection, swin
 from jigsaw_amd.halo import HaloGeometry
 
 pytestmark = pytest.mark.gpu
@@ -119,6 +119,51 @@ def test_hooks_of_saved_tensors_see_what_a_native_node_keeps(kind, dev, monkeypa
     assert len(packed) >= 2
     for a, b in zip(here, want, strict=True):
         assert torch.equal(a, b)
+
+
+def other_layers(dev):
+    """(name, call, leaves) of what has a function of its own beside those of ``layer``."""
+    gen = torch.Generator(device=dev).manual_seed(6)
+    rand = lambda *shape: torch.randn(*shape, device=dev, generator=gen).bfloat16()  # noqa: E731
+
+    def autocast(call):
+        def under(*a):
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                return call(*a)
+        return under
+
+    block = swin.SwinBlock(64, 2, 8, (16, 24), device=dev, one_node=False)
+    norm = lambda x, w, b: layernorm.layer_norm(x, w, b, Half())  # noqa: E731
+    groups = lambda x, w, b: groupnorm.group_norm(x, 3, w, b)  # noqa: E731
+    return [
+        ("linear", projection.linear, [rand(2, 33, 64), rand(48, 64), rand(48)]),
+        ("mlp", projection.gelu_mlp, [rand(40, 64), rand(128, 64), rand(128), rand(64, 128), rand(64)]),
+        ("heads on top of rows", projection.heads_projection_add, [rand(2, 2, 32, 32), rand(64, 64), rand(64), rand(2, 32, 64)]),
+        ("rows that one rank holds", layernorm.plain_layer_norm, [rand(5, 64), rand(64), rand(64)]),
+        ("LayerNorm under autocast", autocast(norm), [rand(5, 7, 72), rand(72).float(), rand(72).float()]),
+        ("all of LayerNorm's results", lambda x, w, b: layernorm._LayerNorm.apply(x, w, b, Half(), 1e-5)[0], [rand(5, 7, 72), rand(72), rand(72)]),
+        ("GroupNorm under autocast", autocast(groups), [rand(2, 12, 9, 11), rand(12).float(), rand(12).float()]),
+        ("all of GroupNorm's results", lambda x, w, b: groupnorm._GroupNorm.apply(x, 3, w, b, (), 1e-5)[0], [rand(2, 12, 9, 11), rand(12), rand(12)]),
+        ("window attention", attention.window_attention, [rand(2, 2, 64, 32), rand(2, 2, 64, 32), rand(2, 2, 64, 32)]),
+        ("block of its parts", autocast(block), [rand(1, 16, 24, 64)]),
+    ]
+
+
+@pytest.mark.parametrize("n", range(10))
+def test_hooks_that_hand_back_another_layout_change_no_gradient(n, dev):
+    name, call, leaves = other_layers(dev)[n]
+    leaves = [t.requires_grad_() for t in leaves]
+
+    def gradients():
+        y = call(*leaves)
+        g = torch.randn(y.shape, device=dev, generator=torch.Generator(device=dev).manual_seed(8)).to(y.dtype)
+        return torch.autograd.grad(y, leaves, g)
+
+    want = gradients()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: torch.stack([t, t], -1)[..., 0]):
+        got = gradients()
+    for a, b in zip(got, want, strict=True):
+        assert torch.equal(a, b), name
 
 
 @pytest.mark.parametrize("kind", KINDS)
