@@ -40,15 +40,19 @@ def layer(kind, dev, back=None, group=None):
     """(call, differentiable tensors, name of the node) of one layer; its input first, its weight second."""
     group = group or Half()
     gen = torch.Generator(device=dev).manual_seed(3)
-    rand = lambda *shape: torch.randn(*shape, device=dev, generator=gen).bfloat16()  # noqa: E731
-    if kind == "conv":
-        size, k, one = (20, 36), (3, 3), (1, 1)
-        geom = HaloGeometry.for_conv(size, k, one, one, one, one, (3, 3))
-        strips = {v: {o: rand(2, 12, *geom.strip_extent(o, v)) for o in itertools.product((-1, 0, 1), repeat=2) if any(o)} for v in ("assemble", "fold")}
-        leaves = [rand(2, 12, *size), rand(24, 12, 3, 3), rand(24)]
-        cfg = conv.HipConvNdConfig.for_rank(2, leaves[2], Exchange(strips["assemble"], back or strips["fold"]))
-        groups = (conv.TileGroup(3, 1),) * 2
-        return (lambda x, w, b: conv._ConvNd.apply(x, w, b, one, one, one, groups, None, cfg)[0]), leaves, "ConvNd"
+    rand = lambda *shape: torch.randn(*shape, device=dev, generator=gen).to(dtype)  # noqa: E731
+    size, stride, dtype = {"conv": ((20, 36), 1, torch.bfloat16), "conv of stride 2": ((20, 36), 2, torch.float16),
+                           "conv of a volume": ((8, 10, 12), 1, torch.float32)}.get(kind, ((), 1, torch.bfloat16))
+    if size:
+        n = len(size)
+        k, one, s = (3,) * n, (1,) * n, (stride,) * n
+        geom = HaloGeometry.for_conv(size, k, s, one, one, one, (3,) * n)
+        strips = {v: {o: rand(2, 12, *e) for o in itertools.product((-1, 0, 1), repeat=n) if any(o) and all(e := geom.strip_extent(o, v))}
+                  for v in ("assemble", "fold")}
+        leaves = [rand(2, 12, *size), rand(24, 12, *k), rand(24)]
+        cfg = conv.HipConvNdConfig.for_rank(n, leaves[2], Exchange(strips["assemble"], back or strips["fold"]))
+        groups = (conv.TileGroup(3, 1),) * n
+        return (lambda x, w, b: conv._ConvNd.apply(x, w, b, s, one, one, groups, None, cfg)[0]), leaves, "ConvNd"
     if kind == "layernorm":
         return (lambda x, w, b: layernorm.layer_norm(x, w, b, group)), [rand(5, 7, 72), rand(72), rand(72)], "LayerNorm"
     if kind == "groupnorm":
@@ -68,7 +72,7 @@ def layer(kind, dev, back=None, group=None):
     return call, [rand(1, 16, 24, 64), *(p.detach().clone() for p in block.parameters())], "WholeBlock"
 
 
-NATIVE = ["conv", "layernorm", "groupnorm"]
+NATIVE = ["conv", "conv of stride 2", "conv of a volume", "layernorm", "groupnorm"]
 KINDS = [*NATIVE, "qkv", "heads", "swin"]
 
 
@@ -81,7 +85,7 @@ def steps(kind, dev, need, monkeypatch, native, hooks=False):
     if not native:
         for module in (conv, layernorm, groupnorm):
             monkeypatch.setattr(module, "native_nodes", lambda: False)
-    leaves = [t.clone().requires_grad_(need[min(i, 1)]) for i, t in enumerate(leaves)]
+    leaves = [t.clone().requires_grad_(need[min(i, len(need) - 1)]) for i, t in enumerate(leaves)]
     packed = []
     if hooks:  # what comes back is laid out otherwise
         with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.shape) or t, lambda t: torch.stack([t, t], -1)[..., 0]):
@@ -101,7 +105,7 @@ def steps(kind, dev, need, monkeypatch, native, hooks=False):
     return [y.detach(), *once], is_native(y), packed
 
 
-@pytest.mark.parametrize("need", [(True, True), (True, False), (False, True)])
+@pytest.mark.parametrize("need", [n for n in itertools.product((True, False), repeat=3) if any(n)], ids=lambda n: "".join(c for c, on in zip("xwb", n) if on))
 @pytest.mark.parametrize("kind", NATIVE)
 def test_a_native_node_has_the_bits_of_the_python_function(kind, need, dev, monkeypatch):
     here, native, _ = steps(kind, dev, need, monkeypatch, True)
@@ -241,3 +245,11 @@ def test_the_collector_frees_a_result_that_its_exchange_keeps(kind, dev):
     del call, leaves, group, keeper
     gc.collect()
     assert gone() is None
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_wrapper_that_a_transform_left_behind_is_taken(kind, dev):
+    call, leaves, _ = layer(kind, dev)
+    left = []
+    torch.func.grad(lambda t: (left.append(t), t.float().sum())[1])(leaves[0])
+    assert torch.equal(call(left[0], *leaves[1:]), call(*leaves))
