@@ -6,6 +6,8 @@ import torch
 from torch import _functorch
 from torch.autograd import forward_ad
 
+from . import _lib
+
 
 def native_nodes() -> bool:
     """Whether a :class:`NativeFunction` may stand for a layer's own autograd function: not under a functorch transform or
@@ -41,20 +43,29 @@ class PositionalFunction(torch.autograd.Function):
 
 class NativeFunction(torch.autograd.Function):
     """The node behind a result that the native host module has computed already: ``apply(result, saved, rest, *inputs)``
-    hands ``result`` out with ``backward(ctx, grad)`` of the subclass behind it, which finds the tensors ``saved`` in
-    ``ctx.saved_tensors`` and ``rest`` as it was given, and returns ``(None, None, None, *gradients of inputs)``.
+    hands ``result`` out with the module's function ``entry`` as its backward, which finds the tensors ``saved`` and ``rest``
+    in the context. Without ``zeros`` an output that nobody used comes as ``None``.
 
-    What it saves on a layer's own function is that function's ``forward`` and ``setup_context``: of steps that wait for the host 10 us
-    in 121 (convolution), 8 in 104 (GroupNorm) and 5 in 118 (sharded LayerNorm). The node is a Python function's all the same, so that
-    the collector sees what it keeps (an exchange that keeps the result makes a cycle through it) and compiled autograd can
-    record it; a node in C++ takes 15 to 20 us less and can do neither. Projections and Swin block gain nothing from it."""
+    The node is a Python function's like any other: the collector sees what it keeps (an exchange that keeps the result makes
+    a cycle through it), and compiled autograd can record it. A node of a C++ class offers neither. What it leaves out is Python on the way: a layer's own ``forward`` and ``setup_context``, and all of the
+    backward, which the engine calls on a thread of its own. Of steps that wait for the host, us on the layer's own function
+    : here (: a node in C++): convolution 118 : 102 (: 94), sharded LayerNorm 116 : 100 (: 92), GroupNorm 100 : 74 (: 62, two launches less among
+    both), projections 87 : 83 (: 78). The Swin block's 340 stay with it."""
+
+    entry = ""
+    zeros = True
 
     @classmethod
     def apply(cls, result, saved, rest, *inputs):
-        return super(torch.autograd.Function, cls).apply((result,), saved, rest, *inputs)
+        if "apply" not in cls._backward_cls.__dict__:
+            # the engine calls a context's ``apply``, compiled autograd the class's ``backward``
+            cls.backward = cls._backward_cls.apply = getattr(_lib.host(), cls.entry)
+        return super(torch.autograd.Function, cls).apply((result,), saved, rest, cls.zeros, *inputs)
 
     @staticmethod
-    def forward(ctx, result, saved, rest, *inputs):  # noqa: D102
+    def forward(ctx, result, saved, rest, zeros, *inputs):  # noqa: D102
         ctx.save_for_backward(*saved)
         ctx.rest = rest
+        if not zeros:
+            ctx.set_materialize_grads(False)
         return result[0]

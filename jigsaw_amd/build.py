@@ -102,8 +102,9 @@ def _compile_host(force: bool) -> Path:
     if not force and _newer(obj, [src, ROOT.parent / "include" / "jigsaw_hip.h"]):
         return obj
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", "-DTORCH_EXTENSION_NAME=_host",
-           "-DTORCH_API_INCLUDE_EXTENSION_H", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
-    for path in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"]):
+           "-DTORCH_API_INCLUDE_EXTENSION_H", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM"]  # (for the stream's type in c10/hip)
+    for path in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"], str(Path(hipcc()).resolve().parent.parent / "include")):
         cmd += ["-isystem", path]
     _run([*cmd, "-c", str(src), "-o", str(obj)], "g++ host.cpp")
     return obj
@@ -115,7 +116,7 @@ def _link_host(obj: Path) -> None:
     cmd = ["g++", "-shared", "-o", str(HOST), str(obj), f"-L{LIB.parent}", "-ljigsaw_hip", "-Wl,-rpath,$ORIGIN/lib"]
     for path in cpp_extension.library_paths():
         cmd += [f"-L{path}", f"-Wl,-rpath,{path}"]
-    _run([*cmd, "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python"], "link of _host.so")
+    _run([*cmd, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"], "link of _host.so")
 
 
 def build(jobs: int = 8, force: bool = False, extra: list[str] | None = None) -> Path:

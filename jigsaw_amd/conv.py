@@ -1072,25 +1072,11 @@ def conv_halo_nway(x, w, b, stride, padding, dilation, spatial_groups, channel_g
     return y, x_aug
 
 
-def _backward_by_plan(step, g, x_aug, weight, stride, padding, dilation, local_in_spatial, spatial_groups, config, need):
-    """``(g_x, g_w, g_b)`` of a layer that the native plan ``step`` runs, or ``None`` where it does not take these tensors."""
-    need_x, need_w, need_b = need
-    stream = _lib.stream_handle(g.device)
-    parts = step.backward(g, x_aug, weight, need_x, need_w, need_w and need_b, stream)
-    if parts is None:
-        return None
-    part, g_w, g_b, send, folded, left = parts
-    if need_b and g_b is None:
-        g_b = config.grad_bias(g.contiguous())
-    if not need_x:
-        return None, g_w, g_b
-    recv = config.halo_exchange.backward(send) if step.sends else {}
-    g_x = step.finish(part, folded, recv, stream, left)
-    if g_x is None:  # strips in another layout
-        ranks, sizes = _mesh_position(spatial_groups)
-        geom = HaloGeometry.for_conv(local_in_spatial, weight.shape[-config.n_spatial :], stride, padding, dilation, ranks, sizes)
-        g_x = halo_fold_border_(part, recv, geom) if folded else halo_fold(part, recv, geom)
-    return g_x, g_w, g_b
+def _fold_without_plan(part, folded, recv, weight, local_in_spatial, stride, padding, dilation, spatial_groups, channel_group, config):
+    """The last step of the backward where the neighbours' strips are not what the native plan takes."""
+    ranks, sizes = _mesh_position(spatial_groups)
+    geom = HaloGeometry.for_conv(local_in_spatial, weight.shape[-config.n_spatial :], stride, padding, dilation, ranks, sizes)
+    return halo_fold_border_(part, recv, geom) if folded else halo_fold(part, recv, geom)
 
 
 def conv_halo_nway_backward(
@@ -1114,11 +1100,18 @@ def conv_halo_nway_backward(
     g_w = g_b = None
     if x_tile is None and g.is_cuda and x_aug.dtype == g.dtype and not getattr(x_aug, "_jg_frame_only", False):
         step = _step_for(config, (*x_aug.shape[:2], *local_in_spatial), x_aug, weight, stride, padding, dilation, ranks, sizes)
-        got = None
-        if step is not None:
-            got = _backward_by_plan(step, g, x_aug, weight, stride, padding, dilation, local_in_spatial, spatial_groups, config, (need_x, need_w, need_b))
-        if got is not None:
-            g_x, g_w, g_b = got
+        stream = _lib.stream_handle(g.device) if step is not None else 0
+        parts = step.backward(g, x_aug, weight, need_x, need_w, need_w and need_b, stream) if step is not None else None
+        if parts is not None:
+            part, g_w, g_b, send, folded, left = parts
+            if need_b and g_b is None:
+                g_b = config.grad_bias(g.contiguous())
+            if not need_x:
+                return done(None)
+            recv = config.halo_exchange.backward(send) if step.sends else {}
+            g_x = step.finish(part, folded, recv, stream, left)
+            if g_x is None:
+                g_x = _fold_without_plan(part, folded, recv, weight, local_in_spatial, stride, padding, dilation, spatial_groups, channel_group, config)
             return done(g_x)
     local_padding = _local_padding(padding, sizes)
     kwargs = {"stride": stride, "padding": local_padding, "dilation": dilation, "groups": int(getattr(config, "groups_local", 1))}
@@ -1322,24 +1315,17 @@ class _NativeConvNd(NativeFunction):
     """``_ConvNd`` of a layer that the native plan runs as it is: the same launches, less of the host. ``rest`` is the
     plan, ``_ConvNd``'s arguments from ``stride`` on and the extents of the tile."""
 
-    @staticmethod
-    def forward(ctx, *args):  # noqa: D102
-        ctx.set_materialize_grads(False)
-        return NativeFunction.forward(ctx, *args)
+    entry, zeros = "conv_backward", False
 
-    @staticmethod
-    def backward(ctx, g):  # noqa: D102
-        if g is None:
-            return (None,) * 6
-        x_aug, weight = ctx.saved_tensors
-        step, (stride, padding, dilation, spatial_groups, channel_group, config), local = ctx.rest
-        need = ctx.needs_input_grad[3:]
-        got = _backward_by_plan(step, g, x_aug, weight, stride, padding, dilation, local, spatial_groups, config, need)
-        if got is None:  # hooks of the saved tensors have given them another layout or type
-            if x_aug.dtype != weight.dtype:
-                x_aug = x_aug.to(weight.dtype)
-            got = conv_halo_nway_backward(g, x_aug, weight, stride, padding, dilation, local, spatial_groups, channel_group, config, need=need)
-        return None, None, None, *got
+
+def _backward_without_plan(ctx, g):
+    """The backward of a :class:`_NativeConvNd` whose saved tensors came back in another layout or type."""
+    x_aug, weight = ctx.saved_tensors
+    _, (stride, padding, dilation, spatial_groups, channel_group, config), local = ctx.rest
+    if x_aug.dtype != weight.dtype:
+        x_aug = x_aug.to(weight.dtype)
+    return None, None, None, None, *conv_halo_nway_backward(g, x_aug, weight, stride, padding, dilation, local, spatial_groups, channel_group, config,
+                                                            need=ctx.needs_input_grad[4:])
 
 
 class _ConvNd(PositionalFunction):

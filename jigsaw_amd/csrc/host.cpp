@@ -13,6 +13,7 @@
 //
 // What a Step does not take (a strip of another shape or layout, tensors of mixed types) it declines by returning
 // None before anything is launched; the callers' Python route then names the error or handles the case.
+#include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 
 #include <algorithm>
@@ -760,9 +761,99 @@ class SwinPass {
   int64_t h = 0, w = 0, shift = 0;
 };
 
+// ---- backward(ctx, grad) of the functions of _autograd.NativeFunction. The engine calls them on a thread of its own with no Python function in
+// between: there Python's objects come from the other thread's core one cache line at a time, and a function of 20 lines took 10 us and more.
+uintptr_t current_stream(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(c10::hip::getCurrentHIPStream(t.device().index()).stream()); }
+
+// What a function's ctx holds
+struct Context {
+  explicit Context(const py::object& ctx) : saved(ctx.attr("saved_tensors")), needs(ctx.attr("needs_input_grad")), rest(ctx.attr("rest")) {}
+  // Saved tensor i row-major, as the kernels' pointers take it: hooks may have given it another layout
+  at::Tensor rows(size_t i) const { return saved[i].cast<at::Tensor>().contiguous(); }
+  bool need(size_t i) const { return needs[4 + i].cast<bool>(); }
+  py::tuple saved, needs, rest;
+};
+// The gradients of (result, saved, rest, zeros, x, weight, bias)
+py::tuple gradients(const py::object& x, const py::object& w, const py::object& b) {
+  const py::object none = py::none();
+  return py::make_tuple(none, none, none, none, x, w, b);
+}
+
+// rest: the plan, _ConvNd's arguments from the stride on, the tile's extents
+py::object conv_backward(const py::object& ctx, const py::object& grad) {
+  const py::object none = py::none();
+  if (grad.is_none()) return gradients(none, none, none);
+  const Context c(ctx);
+  const at::Tensor g = grad.cast<at::Tensor>();
+  const py::tuple args = c.rest[1];
+  const py::handle config = args[5];
+  Step& step = c.rest[0].cast<Step&>();
+  const uintptr_t stream = current_stream(g);
+  const bool need_x = c.need(0), need_w = c.need(1), need_b = c.need(2);
+  const py::object got = step.backward(g, c.saved[0].cast<at::Tensor>(), c.saved[1].cast<at::Tensor>(), need_x, need_w, need_w && need_b, stream);
+  if (got.is_none()) return py::module_::import("jigsaw_amd.conv").attr("_backward_without_plan")(ctx, grad);
+  const py::tuple parts = got;
+  const py::object gb = need_b && parts[2].is_none() ? py::object(config.attr("grad_bias")(g.contiguous())) : py::object(parts[2]);
+  if (!need_x) return gradients(none, parts[1], gb);
+  const py::object recv = step.sends() ? py::object(config.attr("halo_exchange").attr("backward")(parts[3])) : py::dict();
+  py::object gx = step.finish(parts[0].cast<at::Tensor>(), parts[4].cast<bool>(), recv, stream, parts[5]);
+  if (gx.is_none()) gx = py::module_::import("jigsaw_amd.conv").attr("_fold_without_plan")(parts[0], parts[4], recv, c.saved[1], c.rest[2], *args);
+  return gradients(gx, parts[1], gb);
+}
+
+// rest: all_reduce(tensor, "avg" | "sum", group), the group, its size, the type of x and of the parameters
+py::object ln_backward(const py::object& ctx, const py::object& grad) {
+  const py::object none = py::none();
+  if (grad.is_none()) return gradients(none, none, none);
+  const Context c(ctx);
+  const at::Tensor x_norm = c.rows(0), w = c.rows(1), std = c.rows(2), g = grad.cast<at::Tensor>().to(x_norm.scalar_type()).contiguous();
+  const py::object& reduce = c.rest[0];
+  const int64_t ranks = c.rest[2].cast<int64_t>();
+  const uintptr_t stream = current_stream(g);
+  const py::object got = ln_partial_bwd(g, x_norm, w, std, c.need(1), c.need(2), c.rest[4].cast<at::ScalarType>(), stream);
+  TORCH_CHECK(!got.is_none(), "layer_norm: what the backward got is not what the forward saved");
+  const py::tuple parts = got;
+  if (!c.need(0)) return gradients(none, parts[2], parts[3]);
+  if (ranks > 1) {
+    reduce(parts[0], "avg", c.rest[1]);
+    reduce(parts[1], "sum", c.rest[1]);
+  }
+  const at::Tensor gx = ln_bwd_apply(g, x_norm, w, parts[0].cast<at::Tensor>(), parts[1].cast<at::Tensor>(), std, x_norm.size(-1) * ranks, stream);
+  return gradients(py::cast(gx.to(c.rest[3].cast<at::ScalarType>())), parts[2], parts[3]);
+}
+
+// rest: the number of groups, the type of the parameters
+py::object gn_output_backward(const py::object& ctx, const at::Tensor& grad) {
+  const Context c(ctx);
+  const at::Tensor x = c.rows(0);
+  const at::Tensor g = grad.to(x.scalar_type()).contiguous();
+  const c10::optional<at::Tensor> w = c.saved[3].is_none() ? c10::nullopt : c10::optional<at::Tensor>(c.rows(3));
+  const py::object got = gn_backward(g, x, c.rows(1), c.rows(2), w, c.rest[0].cast<int64_t>(), c.need(0), c.need(1), c.need(2),
+                                     c.rest[1].cast<at::ScalarType>(), current_stream(g));
+  TORCH_CHECK(!got.is_none(), "group_norm: what the backward got is not what the forward saved");
+  const py::tuple all = got;
+  return gradients(all[0], all[1], all[2]);
+}
+
+// rest: projection_backward, whether it is the qkv projection's, batch, heads, tokens and columns of a head
+py::object projection_node_backward(const py::object& ctx, const at::Tensor& grad) {
+  const Context c(ctx);
+  const at::Tensor g = grad.contiguous();
+  const py::object got = c.rest[0](g, c.rows(0), c.rows(1), c.rest[1], c.rest[2], c.rest[3], c.rest[4], c.rest[5], c.need(0), c.need(1), c.need(2), current_stream(g));
+  TORCH_CHECK(!got.is_none(), "projection: what the backward got is not what the forward saved");
+  const py::tuple all = got;
+  return gradients(all[0], all[1], all[2]);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  // functions that a class may hold as methods
+  auto method = [&](const char* name, auto f) { m.attr(name) = py::cpp_function(f, py::name(name), py::is_method(py::none())); };
+  method("conv_backward", &conv_backward);
+  method("ln_backward", &ln_backward);
+  method("gn_output_backward", &gn_output_backward);
+  method("projection_node_backward", &projection_node_backward);
   py::class_<SumsLeft>(m, "SumsLeft");
   py::class_<Step>(m, "Step")
       .def(py::init<const py::tuple&, const py::tuple&, const py::tuple&, const py::tuple&, int, int, uintptr_t, uintptr_t, bool,

@@ -265,15 +265,7 @@ class _NativeGroupNormOutput(NativeFunction):
     """``_GroupNormOutput`` of a tensor that one rank holds whole, in the type that it is computed in, by the native host
     module: the same launches, less of the host."""
 
-    @staticmethod
-    def backward(ctx, g):  # noqa: D102
-        x, mean, rstd, w = saved_rows(ctx)
-        groups, grad_dtype = ctx.rest
-        got = _lib.host().gn_backward(g.to(x.dtype).contiguous(), x, mean, rstd, w, groups, *ctx.needs_input_grad[3:], grad_dtype,
-                                      _lib.stream_handle(g.device))
-        if got is None:
-            raise RuntimeError("group_norm: what the backward got is not what the forward saved")
-        return None, None, None, *got
+    entry = "gn_output_backward"
 
 
 def group_norm(x, num_groups, weight=None, bias=None, spatial_groups=(), eps=1e-5):

@@ -64,24 +64,6 @@ def _compute_dtype(x: torch.Tensor) -> torch.dtype:
     return x.dtype
 
 
-def _native_backward(g, x_norm, w, std, need, grad_dtype, group):
-    """Gradients of the input (in ``g``'s type), the weight and the bias (in ``grad_dtype``) by the native host module, or ``None``."""
-    host = _lib.host()
-    if host is None:
-        return None
-    handle = _lib.stream_handle(g.device)
-    parts = host.ln_partial_bwd(g, x_norm, w, std, need[1], need[2], grad_dtype, handle)
-    if parts is None:
-        return None
-    mean_gxn, dot, gw, gb = parts
-    grad_x = None
-    if need[0]:
-        _all_reduce(mean_gxn, "avg", group)
-        _all_reduce(dot, "sum", group)
-        grad_x = host.ln_bwd_apply(g, x_norm, w, mean_gxn, dot, std, x_norm.shape[-1] * _group_size(group), handle)
-    return grad_x, gw, gb
-
-
 class _LayerNorm(PositionalFunction):
     """Autograd function of the distributed LayerNorm (HIP kernels inside)."""
 
@@ -163,10 +145,18 @@ class _LayerNorm(PositionalFunction):
         # the column sums leave the kernel in the parameters' dtype where they share one
         wdt, bdt = ctx.param_dtypes
         gdt = wdt if wdt in _lib._DTYPES and bdt in (None, wdt) else torch.float32
-        got = _native_backward(g, x_norm, w, std, (need_x, need_w, need_b), gdt, group)
-        if got is not None:  # the same calls as below
-            grad_x, gw, gb = got
-            return (grad_x.to(ctx.in_dtype) if need_x else None), (gw.to(wdt) if need_w else None), (gb.to(bdt) if need_b else None), None, None
+        host = _lib.host()
+        if host is not None:  # the same calls as below
+            handle = _lib.stream_handle(dev)
+            parts = host.ln_partial_bwd(g, x_norm, w, std, need_w, need_b, gdt, handle)
+            if parts is not None:
+                mean_gxn, dot, gw, gb = parts
+                grad_x = None
+                if need_x:
+                    _all_reduce(mean_gxn, "avg", group)
+                    _all_reduce(dot, "sum", group)
+                    grad_x = host.ln_bwd_apply(g, x_norm, w, mean_gxn, dot, std, n_global, handle).to(ctx.in_dtype)
+                return grad_x, (gw.to(wdt) if need_w else None), (gb.to(bdt) if need_b else None), None, None
 
         lib = _lib.load()
         mean_gxn, dot = torch.empty((2, *std.shape), dtype=torch.float32, device=dev).unbind(0)
@@ -200,22 +190,7 @@ class _NativeLayerNorm(NativeFunction):
     """``_LayerNorm`` for the caller of :func:`layer_norm` with parameters in the type that ``y`` gets, by the native host module
     alone: the same launches, less of the host."""
 
-    @staticmethod
-    def forward(ctx, *args):  # noqa: D102
-        ctx.set_materialize_grads(False)
-        return NativeFunction.forward(ctx, *args)
-
-    @staticmethod
-    def backward(ctx, g):  # noqa: D102
-        if g is None:
-            return (None,) * 6
-        x_norm, w, std = saved_rows(ctx)
-        group, in_dtype, grad_dtype = ctx.rest
-        need = ctx.needs_input_grad[3:]
-        got = _native_backward(g.to(x_norm.dtype).contiguous(), x_norm, w, std, need, grad_dtype, group)
-        if got is None:
-            raise RuntimeError("layer_norm: what the backward got is not what the forward saved")
-        return None, None, None, got[0].to(in_dtype) if need[0] else None, got[1], got[2]
+    entry, zeros = "ln_backward", False
 
 
 def layer_norm(x, weight, bias, channel_group=None, eps: float = 1e-5) -> torch.Tensor:
@@ -234,7 +209,7 @@ def layer_norm(x, weight, bias, channel_group=None, eps: float = 1e-5) -> torch.
     y, x_norm, _ = host.ln_apply(x, mean, var, std, weight, bias, float(eps), handle)
     if not wants_grad(x, weight, bias):
         return y
-    return _NativeLayerNorm.apply(y, (x_norm, weight, std), (channel_group, x.dtype, weight.dtype), x, weight, bias)
+    return _NativeLayerNorm.apply(y, (x_norm, weight, std), (_all_reduce, channel_group, ranks, x.dtype, weight.dtype), x, weight, bias)
 
 
 class _PlainLayerNorm(torch.autograd.Function):

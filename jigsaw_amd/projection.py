@@ -25,7 +25,7 @@ import math
 import torch
 
 from . import _lib
-from ._autograd import saved_rows
+from ._autograd import NativeFunction, native_nodes, saved_rows, wants_grad
 
 
 def _nt(out, a, w, bias, rows, n_out, k_in, a_heads, out_heads, dims) -> None:
@@ -188,6 +188,33 @@ def _native(*tensors):
     """The native host module where it may take these tensors (parameters in the tokens' type, so that there is nothing to
     cast or to remember), else ``None``."""
     return _lib.host() if all(t is None or (t.is_cuda and t.dtype == tensors[0].dtype) for t in tensors) else None
+
+
+class _NativeQkvProjection(NativeFunction):
+    """``_QkvProjection`` where forward and backward are the native host module's."""
+
+    entry = "projection_node_backward"
+
+
+class _NativeHeadsProjection(NativeFunction):
+    """``_HeadsProjection`` where forward and backward are the native host module's."""
+
+    entry = "projection_node_backward"
+
+
+def _native_apply(x, weight, bias, heads: int | None):
+    """The qkv projection, or the heads projection where ``heads`` is ``None``, by the native host module alone, or ``None``."""
+    host = _native(x, weight, bias) if not _remember_casts and native_nodes() else None
+    if host is None:
+        return None
+    qkv, stream = heads is not None, _lib.stream_handle(x.device)
+    y = host.qkv_forward(x, weight, bias, heads, stream) if qkv else host.heads_forward(x, weight, bias, stream)
+    if y is None or not wants_grad(x, weight, bias):
+        return y
+    split = y if qkv else x
+    h, s, d = split.shape[-3:]
+    rest = (host.projection_backward, qkv, x.numel() // (x.shape[-1] * s * (1 if qkv else h)), h, s, d)
+    return (_NativeQkvProjection if qkv else _NativeHeadsProjection).apply(y, (x, weight), rest, x, weight, bias)
 
 
 def _native_backward(ctx, grad, x, w, qkv: bool):
@@ -471,12 +498,18 @@ def gelu_mlp(x, w1, b1, w2, b2, residual=None):
 def qkv_projection(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, heads: int) -> torch.Tensor:
     """``rearrange(F.linear(x, weight, bias), "... s (three h d) -> three ... h s d", three=3, h=heads)``
     without the intermediate ``(..., s, 3 h d)`` tensor (_attention.py:881-890)."""
+    y = _native_apply(x, weight, bias, heads)
+    if y is not None:
+        return y
     return _QkvProjection.apply(x, weight, bias, heads)
 
 
 def heads_projection(out: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """``F.linear(rearrange(out, "... h s d -> ... s (h d)"), weight, bias)`` without the
     contiguous copy of the rearranged tensor (_attention.py:909-916)."""
+    y = _native_apply(out, weight, bias, None)
+    if y is not None:
+        return y
     return _HeadsProjection.apply(out, weight, bias, None)
 
 

@@ -72,8 +72,8 @@ def layer(kind, dev, back=None, group=None):
     return call, [rand(1, 16, 24, 64), *(p.detach().clone() for p in block.parameters())], "WholeBlock"
 
 
-NATIVE = ["conv", "conv of stride 2", "conv of a volume", "layernorm", "groupnorm"]
-KINDS = [*NATIVE, "qkv", "heads", "swin"]
+NATIVE = ["conv", "conv of stride 2", "conv of a volume", "layernorm", "groupnorm", "qkv", "heads"]
+KINDS = [*NATIVE, "swin"]
 
 
 def is_native(y):
@@ -83,7 +83,7 @@ def is_native(y):
 def steps(kind, dev, need, monkeypatch, native, hooks=False):
     call, leaves, name = layer(kind, dev)
     if not native:
-        for module in (conv, layernorm, groupnorm):
+        for module in (conv, layernorm, groupnorm, projection):
             monkeypatch.setattr(module, "native_nodes", lambda: False)
     leaves = [t.clone().requires_grad_(need[min(i, len(need) - 1)]) for i, t in enumerate(leaves)]
     packed = []
