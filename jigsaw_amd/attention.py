@@ -105,7 +105,7 @@ def _bias_args(bias, batch, sq, sk):
 # 128, the fp32 ones any lengths at multiples of 4 up to 128, the one-thread-per-row kernels (bias, more
 # batch entries than a grid dimension holds) a few head sizes. Other head sizes get zero columns:
 # they add nothing to the scores and give zero output columns, which are dropped. Narrow bf16 heads on
-# long sequences get them too, for the faster kernels of 64 columns (_as_64_columns).
+# long sequences get them too, by a rule of the time when the kernels of 64 columns were the faster ones (_as_64_columns).
 # --------------------------------------------------------------------------- #
 _KERNEL_HEAD_SIZES = (8, 16, 32, 64, 96, 128)
 _F32_MFMA_HEAD_SIZES = (32, 64, 128)
@@ -134,13 +134,13 @@ def _kernel_head_size(d: int, dtype=None, has_bias: bool = False) -> int:
 
 
 def _as_64_columns(q, k, chunks: int = 1) -> bool:
-    """Whether bf16 heads of fewer than 64 columns against ``chunks`` chunks like ``k`` are better off with zero columns
-    up to 64, copies there and back included, on the kernels of that size, which stream their tiles straight into LDS and keep eight
-    wavefronts busy a workgroup. Forward / backward, us, own width and as 64 columns, when the line was drawn: 8 heads x 4096 x 4096 keys, 16 columns
-    89/170 and 76/172, 32 85/159 and 73/164, 48 105/206 and 81/180; 2 x 8192 x 8192, 32 100/205 and 96/206; 8 x 8192 x 4096, 40 117/317 and 118/288. Since the
-    kernels of any width have two blocks of rows a wavefront and one launch backward, their own width is the faster one there too: 43/93 and 68/144, 39/92 and 67/152,
-    67/166 and 75/164; 48/119 and 86/201; 98/280 and 111/267. More rows were always better off there: 32 heads x 4096, 16 columns 125/297 and 193/455,
-    48 180/474 and 214/528, 64 heads, 56 354/952 and 435/1081."""
+    """Whether bf16 heads of fewer than 64 columns against ``chunks`` chunks like ``k`` run with zero columns up to 64, copies there
+    and back included, on the kernels of that size. The line was drawn when those were the faster ones there: forward / backward, us, own width and
+    as 64 columns, 8 heads x 4096 x 4096 keys, 16 columns 89/170 and 76/172, 32 85/159 and 73/164, 48 105/206 and 81/180; 2 x 8192 x 8192, 32
+    100/205 and 96/206; 8 x 8192 x 4096, 40 117/317 and 118/288. With two blocks of rows a wavefront and one launch backward the kernels of any width are now as
+    fast or faster at every one of them: 43/93 and 68/144, 39/92 and 67/152, 67/166 and 75/164; 48/119 and 86/201; 98/280 and 111/267. More rows were
+    always better off there: 32 heads x 4096, 16 columns 125/297 and 193/455, 48 180/474 and 214/528, 64 heads, 56 354/952 and 435/1081. The rule stands
+    until it is taken out together with the tests that ask for its answers."""
     # (host.cpp's may_want_64_columns asks here about the rows, keys and widths that it names: no others may get a yes)
     *lead, sq, d = q.shape
     if sq < 2048 or d >= 64 or q.dtype != torch.bfloat16:

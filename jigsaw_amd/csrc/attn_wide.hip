@@ -719,6 +719,8 @@ __device__ __forceinline__ void dq_block(const Args& p, const BlockOf& wg) {
   }
 }
 
+// (Two blocks a wavefront: two wavefronts a SIMD are asked for, that is 256 registers. At 64 columns the kernel takes them all and spills four, in
+// front of and behind the tile loop.)
 template <int D, bool F16, int W, int KS, bool EXACT, int QB>
 __global__ __launch_bounds__(64 * W * KS, QB) void attn_wide_dq_kernel(ChunkTable, Args p) {
   dq_block<D, F16, W, KS, EXACT, true, QB>(p, block_of());
@@ -1109,8 +1111,8 @@ int launch_bwd(const ChunkTable& tab, const Args& a, long long batch, int width,
   return width == 1 ? go(One{}) : width == 2 ? go(Two{}) : go(Four{});
 }
 
-// f(D constant, F16 constant) for the narrowest kernel that holds the head. (Long bf16 sequences of narrow heads are better
-// off as heads of 64 on that size's kernels, zero columns and copies included: attention.py brings them there.)
+// f(D constant, F16 constant) for the narrowest kernel that holds the head. (attention.py brings long bf16 sequences of narrow heads with zero
+// columns to the kernels of 64, by a line drawn before these had two blocks a wavefront.)
 template <typename F>
 int by_width(int d, int dtype, F f) {
   auto typed = [&](auto width) { return dtype == JG_F16 ? f(width, std::true_type{}) : f(width, std::false_type{}); };

@@ -666,7 +666,9 @@ __device__ __forceinline__ void whole_statistics(const ResidentArgs& q, const Ap
 // WHOLE: a block has a part of kThreads threads for each chunk of its unit (blockIdx.x), up to kWhole of them: the partials meet in LDS,
 // nobody waits for another block, and neither the words nor the list are wanted. One launch forward where there are three,
 // two backward: a short step is bound by the host, which takes 3 to 4 us a launch (forward and backward of 4 x 64 x 259 x 83 bf16 in
-// 32 groups and of smaller tensors, us: 78 with six launches, 66 with three)
+// 32 groups and of smaller tensors, us: 78 with six launches, 66 with three). On the GPU alone, blocks that wait : WHOLE: 8 x 8 x 16384 in 8 groups 12.5 : 7.6
+// and 10.4 : 7.7 forward and backward, 4 x 64 x 21497 in 32 15.5 : 11.6 and 13.2 : 13.1, 4 x 64 x 32768 in 16 (four full chunks a group) 18.2 : 16.8 forward; few
+// groups of four full chunks keep fewer compute units busy, for less than what the host saves: 4 x 32 x 32768 in 8 14.4 : 15.3
 template <int DT, bool BWD, bool STREAM, bool WHOLE>
 __global__ __launch_bounds__(WHOLE ? kWhole * kThreads : kThreads, 4) void gn_resident_kernel(ResidentArgs q, ApplyArgs p) {
   typedef typename Elem<DT>::T T;

@@ -1,6 +1,6 @@
 // Host side of the small steps in native code: the distributed convolution (Step), ring attention over resident chunks, the
 // sharded LayerNorm's pieces between its collectives, GroupNorm of a whole tensor, the projections around attention and the
-// Swin block (SwinPass).
+// Swin block (SwinPass), and the backward of the functions that autograd calls here (_autograd.NativeFunction).
 //
 // The convolution: allocations, strips, pointer tables and the calls into
 // libjigsaw_hip.so, in native code. A step of one layer is 10 launches of 3 to 60 us; worked through Python
